@@ -648,11 +648,18 @@ int spx_gemm_bf16_tn_f32(const void* a, int64_t lda, const void* b, int64_t ldb,
  * e * b_group_stride ([N, K], row stride ldb).  The workspace (spx_gemm_grouped_workspace_bytes,
  * 4-byte aligned) holds the tile table the launch builds on the device.  Same operand rules as
  * spx_gemm_bf16_nt.
+ * spx_gemm_bf16_nn_grouped: the same with b_e as it lies the other way, c[r, :] = a[r, :] * b_e, b_e [K, N]
+ * (row stride ldb): the input gradient of the product above against the same weight stack, with no
+ * transposed copy of it.  N must be a multiple of 8 as well; same workspace.
  * spx_gemm_bf16_tn_grouped: c_e[M, N] (+)= a[rows of e, :M]^T * b[rows of e, :N], c_e = c +
  * e * c_group_stride elements; out_f32 selects an fp32 c; without `accumulate` an empty group
  * gets zeros.  Same operand rules as spx_gemm_bf16_tn. */
 int64_t spx_gemm_grouped_workspace_bytes(int64_t rows, int64_t groups);
 int spx_gemm_bf16_nt_grouped(const void* a, int64_t lda, const void* b, int64_t ldb,
+                             int64_t b_group_stride, void* c, int64_t ldc, int64_t rows,
+                             int64_t N, int64_t K, const int32_t* group_offsets, int64_t groups,
+                             void* workspace, int64_t workspace_bytes, void* stream);
+int spx_gemm_bf16_nn_grouped(const void* a, int64_t lda, const void* b, int64_t ldb,
                              int64_t b_group_stride, void* c, int64_t ldc, int64_t rows,
                              int64_t N, int64_t K, const int32_t* group_offsets, int64_t groups,
                              void* workspace, int64_t workspace_bytes, void* stream);
@@ -680,6 +687,15 @@ int spx_gemm_bf16_tn_grouped_multi(const void* a, int64_t lda, const void* b, in
 int spx_transpose_bf16(const void* in, int64_t ld_in, int64_t batch_stride_in, void* out,
                        int64_t ld_out, int64_t batch_stride_out, int64_t R, int64_t C,
                        int64_t batches, void* stream);
+
+/* The (token, slot) pairs of a router's choice idx (int64 [tokens, k], values 0 .. experts - 1; others are
+ * clamped) sorted by expert, stable: order[r] = pair t * k + j of sorted row r, src_row[r] = its token,
+ * pos[t, j] = its sorted row, offsets[e] .. offsets[e + 1] = the rows of expert e (int32 [experts + 1]).
+ * At most 2048 experts; workspace: spx_moe_sort_workspace_bytes(tokens * k, experts), 4-byte aligned. */
+int64_t spx_moe_sort_workspace_bytes(int64_t pairs, int64_t experts);
+int spx_moe_sort_pairs(const int64_t* idx, int64_t tokens, int32_t k, int64_t experts, int64_t* order,
+                       int32_t* src_row, int32_t* pos, int32_t* offsets, void* workspace,
+                       int64_t workspace_bytes, void* stream);
 
 /* Row movement between the token order [tokens, H] and the expert-sorted order [rows, H] (bf16;
  * index_select / index_add_ of Qwen3NextExperts.forward and their backward):

@@ -29,6 +29,7 @@
 
 #include <type_traits>
 
+#include "gemm_tile_api.h"
 #include "spx_common.h"
 #include "../../include/spx.h"
 
@@ -756,11 +757,6 @@ __global__ __launch_bounds__(256) void gemm_group_tiles_kernel(const int32_t* __
 }
 }  // namespace spx
 
-extern "C" int64_t spx_gemm_grouped_workspace_bytes(int64_t rows, int64_t groups) {
-  if (rows < 0 || groups < 0) return 0;
-  return (int64_t)sizeof(int32_t) * (1 + 2 * ((rows + kTM - 1) / kTM + groups));
-}
-
 extern "C" int spx_gemm_bf16_nt_grouped(const void* a, int64_t lda, const void* b, int64_t ldb,
                                         int64_t b_group_stride, void* c, int64_t ldc, int64_t rows,
                                         int64_t N, int64_t K, const int32_t* group_offsets,
@@ -772,6 +768,12 @@ extern "C" int spx_gemm_bf16_nt_grouped(const void* a, int64_t lda, const void* 
   SPX_REQ_FN(workspace_bytes >= spx_gemm_grouped_workspace_bytes(rows, groups), "workspace too small");
   SPX_REQ_FN(((uintptr_t)workspace) % 4 == 0 && b_group_stride % 8 == 0 && b_group_stride >= 0,
              "unaligned workspace or group stride");
+  // Up to 1536 rows a group on average the 128-row tile of gemm_tile.hip wins: its bands fit the groups better and
+  // two tiles' worth of loads are in flight (80 rows: 573 -> 456 us, 256: 1217 -> 1111, 640: 228 -> 209; 2560 rows
+  // 641 us here against 687 there; gate/up shapes, see gemm_tile.hip)
+  if (rows <= 1536 * groups)
+    return tile::grouped_nt(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups,
+                            workspace, stream);
   int32_t* tab = reinterpret_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(gemm_group_tiles_kernel, dim3(1), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
                      group_offsets, (int)groups, (int)rows, (int)((rows + kTM - 1) / kTM + groups), tab);

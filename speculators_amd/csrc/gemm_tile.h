@@ -1,0 +1,342 @@
+// Small-tile bf16 GEMM kernels for gfx950 (NT, NN and TN forms, plain, cut along the contraction, grouped).
+// Instantiated and launched by gemm_tile.hip.
+#pragma once
+
+#include "spx_common.h"
+
+namespace spx {
+namespace tile {
+
+constexpr int kTK = 64;  // contraction columns per slab
+constexpr int kOob = 0x7ffffff0;
+
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef short i16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ i16x4 read_tr16(uint32_t addr) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(uintptr_t)addr);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// One operand of a tile: kR rows of C (or columns of C) x one slab of 64 contraction indices, staged through LDS.
+// SLOW = false: the contraction index is contiguous in memory (a row of the operand holds it); LDS holds kR rows
+// of 128 bytes, 16-byte chunk c of row r in slot c ^ f(r), f(r) = (r & 7) ^ ((r >> 3) & 1).
+// SLOW = true: the contraction index is the slow one (the operand is stored [contraction, kR columns]); LDS holds
+// 64 rows of 2 kR bytes, 32-byte piece p of row t in position p ^ h(t), h(t) = t % 4 + 4 (t / 8 % 2), and the
+// fragments are taken with the transposing read.
+template <int kR, int kWaves, bool SLOW>
+struct Operand {
+  static constexpr int kBytes = kR * kTK * 2;         // per slab
+  static constexpr int kLoads = kBytes / 1024 / kWaves;  // 1 KB wave-loads per wave and slab
+  static_assert(kBytes % (1024 * kWaves) == 0, "whole wave-loads");
+  u32x4 rsrc;
+  int off[kLoads];
+  int kchunk[SLOW ? 1 : 2];  // first contraction index of this lane's chunk inside the slab (even / odd row groups)
+  int row_bytes;
+
+  // base: the operand's first element of this tile (and contraction range); rows: how many of the kR lie inside the
+  // matrix; len: contraction length
+  __device__ __forceinline__ void init(const uint16_t* base, int64_t ld, int rows, int len, int wave, int lane) {
+    row_bytes = (int)(ld * 2);
+    if (!SLOW) {
+      rsrc = make_rsrc(base, len > 0 && rows > 0 ? (uint32_t)((((int64_t)min(rows, kR) - 1) * ld + len) * 2) : 0u);
+      const int lrow = lane >> 3;
+      const int c0 = (lane & 7) ^ (lrow & 7);
+      kchunk[0] = c0 * 8;
+      if constexpr (!SLOW) kchunk[1] = (c0 ^ 1) * 8;
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const int g = wave * kLoads + j;  // 8-row group
+        const int r = g * 8 + lrow;
+        off[j] = r < rows ? (int)(((int64_t)r * ld + (c0 ^ (g & 1)) * 8) * 2) : kOob;
+      }
+    } else {
+      rsrc = make_rsrc(base, len > 0 && rows > 0 ? (uint32_t)((((int64_t)len - 1) * ld + min(rows, kR)) * 2) : 0u);
+      constexpr int kRow = kR * 2, kPerLoad = 1024 / kRow, kLanes = kRow / 16;
+      const int lrow = lane / kLanes, lpos = lane % kLanes;
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const int r = kPerLoad * (wave * kLoads + j) + lrow;
+        const int hr = ((r & 3) | (((r >> 3) & 1) << 2)) & (kR / 16 - 1);
+        const int c8 = ((((lpos >> 1) ^ hr) << 1) | (lpos & 1)) * 8;
+        off[j] = c8 < rows ? (int)(((int64_t)r * ld + c8) * 2) : kOob;
+      }
+    }
+  }
+
+  // wave-load j of the slab at contraction index k0 into the LDS slab at `lds` (this operand's base)
+  __device__ __forceinline__ void load(int j, uint32_t lds, int k0, int len, int wave) const {
+    const uint32_t dst = lds + (wave * kLoads + j) * 1024;
+    if (!SLOW) {
+      // (a chunk past the end of the contraction would read the next row: its lane goes out of range)
+      const int g = wave * kLoads + j;
+      const int kc = k0 + ((g & 1) ? kchunk[SLOW ? 0 : 1] : kchunk[0]);
+      load_to_lds16<0>(rsrc, dst, kc < len ? off[j] : kOob, k0 * 2);
+    } else {
+      // the whole offset is in the vector register, which is what the range check sees
+      load_to_lds16<0>(rsrc, dst, (int)((uint32_t)off[j] + (uint32_t)k0 * (uint32_t)row_bytes), 0);
+    }
+  }
+
+  // fragment f (16 rows of this wave's stripe, which starts at row w0) of K step kk out of the slab at `lds`
+  __device__ __forceinline__ static uint32_t read_base(uint32_t lds0, int w0, int lane) {
+    const int q = lane >> 4, r16 = lane & 15;
+    if (!SLOW) {
+      const int fr = (r16 & 7) ^ (r16 >> 3);
+      return lds0 + (w0 + r16) * 128 + ((q ^ fr) * 16);
+    }
+    const int trow = 8 * q + (r16 >> 2);
+    return lds0 + trow * (kR * 2) + 8 * (r16 & 3);
+  }
+  __device__ __forceinline__ static bf16x8 read(uint32_t base, uint32_t slab, int w0, int f, int kk, int lane) {
+    if (!SLOW) {
+      union { u32x4 u; bf16x8 b; } c;
+      c.u = lds_read128((base ^ (kk * 64)) + slab + f * 16 * 128);
+      return c.b;
+    }
+    const int q = lane >> 4, r16 = lane & 15;
+    const int h = ((r16 >> 2) | ((q & 1) << 2)) & (kR / 16 - 1);
+    const uint32_t a = base + slab + kk * 32 * (kR * 2) + ((((w0 >> 4) + f) ^ h) * 32);
+    const i16x4 lo = read_tr16(a), hi = read_tr16(a + 4 * (kR * 2));
+    const i16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, v);
+  }
+};
+
+struct Params {
+  const uint16_t* A;
+  const uint16_t* B;
+  void* C;
+  int64_t lda, ldb, ldc;
+  int M, N, K;
+  int tiles_m, tiles_n;
+  int parts;                    // the contraction is cut into this many parts (> 1: fp32 partials in part_ws)
+  float* part_ws;               // [parts][M][N]
+  const int32_t* tile_tab;      // grouped NT / NN: (group, first row) per tile row, see gemm_group_tiles_kernel
+  const int32_t* group_off;     // grouped: group boundaries
+  int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)
+};
+
+// OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT>
+__global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p) {
+  constexpr int kWaves = WM * WN, kMI = TM / WM / 16, kNI = TN / WN / 16;
+  using OA = Operand<TM, kWaves, AT>;
+  using OB = Operand<TN, kWaves, BT>;
+  constexpr int kStage = OA::kBytes + OB::kBytes;
+  constexpr int kL = OA::kLoads + OB::kLoads;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+
+  int M = p.M, K = p.K;
+  const uint16_t *A = p.A, *B = p.B;
+  void* C = p.C;
+  int tiles_m = p.tiles_m;
+  if (!AT && p.tile_tab) tiles_m = min(p.tile_tab[0], tiles_m);
+  const int n_tiles = tiles_m * p.tiles_n, n_wg = n_tiles * p.parts;
+  if ((int)blockIdx.x >= n_wg) return;
+  // one contiguous run of tiles per XCD (workgroups go to the eight XCDs round robin), all parts of a tile in it:
+  // an XCD's tiles share their operand bands in its L2
+  int pid;
+  {
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, base = n_wg >> 3, rem = n_wg & 7;
+    pid = xcd * base + min(xcd, rem) + local;
+  }
+  const int part = pid / n_tiles;
+  pid -= part * n_tiles;
+  int tm, tn;
+  if (!AT && p.tile_tab) {  // grouped: the column tiles of one tile row run together (they share the group's rows)
+    tm = pid / p.tiles_n;
+    tn = pid % p.tiles_n;
+  } else {
+    // groups of four tile rows, columns first inside a group
+    constexpr int kGroup = 4;
+    const int g = pid / (kGroup * p.tiles_n), r = pid % (kGroup * p.tiles_n);
+    const int gs = min(tiles_m - g * kGroup, kGroup);
+    tm = g * kGroup + r % gs;
+    tn = r / gs;
+  }
+  int m0 = tm * TM;
+  const int n0 = tn * TN;
+  if (!AT && p.tile_tab) {
+    const int grp = p.tile_tab[1 + 2 * tm];
+    m0 = p.tile_tab[2 + 2 * tm];
+    M = min(M, max(p.group_off[grp + 1], 0));
+    B += (int64_t)grp * p.group_stride;
+  }
+  if (AT && p.group_off) {  // grouped TN: blockIdx.y = group, the contraction runs over its rows
+    const int e = blockIdx.y;
+    const int t0 = min(max(p.group_off[e], 0), p.K), t1 = min(max(p.group_off[e + 1], t0), p.K);
+    A += (int64_t)t0 * p.lda;
+    B += (int64_t)t0 * p.ldb;
+    K = t1 - t0;
+    C = reinterpret_cast<uint8_t*>(C) + (int64_t)e * p.group_stride * (OUT >= 2 ? 4 : 2);
+    if ((OUT & 1) && K == 0) return;
+  }
+  if (p.parts > 1) {
+    const int slabs = ((K + kTK - 1) / kTK + p.parts - 1) / p.parts;
+    const int k_begin = part * slabs * kTK;
+    A += AT ? (int64_t)k_begin * p.lda : (int64_t)k_begin;
+    B += BT ? (int64_t)k_begin * p.ldb : (int64_t)k_begin;
+    K = max(min(K - k_begin, slabs * kTK), 0);
+  }
+
+  OA oa;
+  OB ob;
+  oa.init(AT ? A + m0 : A + (int64_t)m0 * p.lda, p.lda, M - m0, K, wave, lane);
+  ob.init(BT ? B + n0 : B + (int64_t)n0 * p.ldb, p.ldb, p.N - n0, K, wave, lane);
+  const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+  const uint32_t a_rd = OA::read_base(lds0, wm, lane), b_rd = OB::read_base(lds0 + OA::kBytes, wn, lane);
+
+  f32x4 acc[kNI][kMI];
+#pragma unroll
+  for (int j = 0; j < kNI; ++j)
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nslab = (K + kTK - 1) / kTK;
+  int ld_k = 0;  // contraction index of the slab being loaded
+  uint32_t ld_at = lds0;
+  auto issue_one = [&](int l) __attribute__((always_inline)) {
+    if (l < OA::kLoads) oa.load(l, ld_at, ld_k, K, wave);
+    else ob.load(l - OA::kLoads, ld_at + OA::kBytes, ld_k, K, wave);
+  };
+  auto next_load = [&]() __attribute__((always_inline)) {
+    ld_k += kTK;
+    ld_at = ld_at + kStage == lds0 + STAGES * kStage ? lds0 : ld_at + kStage;
+  };
+  bf16x8 fa[2][kMI], fb[2][kNI];
+  uint32_t rd = 0;  // slab buffer the reads go to
+  auto read_one = [&](int set, int kk, int f) __attribute__((always_inline)) {
+    if (f < kMI) fa[set][f] = OA::read(a_rd, rd, wm, f, kk, lane);
+    else fb[set][f - kMI] = OB::read(b_rd, rd, wn, f - kMI, kk, lane);
+  };
+  // One K step of 32: the products on register set `set`; between them the LDS reads that fill the other set with K
+  // step rk and (loads) the wave-loads of a whole slab
+  auto step = [&](int set, int rk, bool loads) __attribute__((always_inline)) {
+    constexpr int kN = kNI * kMI, kF = kMI + kNI;
+    int reads = 0, issued = 0;
+#pragma unroll
+    for (int j = 0; j < kNI; ++j)
+#pragma unroll
+      for (int i = 0; i < kMI; ++i) {
+        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[set][j], fa[set][i], acc[j][i], 0, 0, 0);
+        const int idx = j * kMI + i;
+        __builtin_amdgcn_sched_barrier(0);
+        // reads in the first three quarters of the step, loads evenly
+        while (reads < kF && reads * kN * 3 < (idx + 1) * kF * 4) { read_one(set ^ 1, rk, reads++); }
+        if (loads)
+          while (issued < kL && issued * kN < (idx + 1) * kL) issue_one(issued++);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+
+  // STAGES slab buffers (past the last slab the loads bring zeros)
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+    for (int l = 0; l < kL; ++l) issue_one(l);
+    next_load();
+  }
+  wait_vmcnt<(STAGES - 1) * kL>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
+  for (int s = 0; s < nslab; ++s) {
+    __builtin_amdgcn_sched_barrier(0);
+    step(0, 1, false);
+    // every read of slab s has returned; after the barrier for every wave (its buffer is free) and slab s + 1 has
+    // landed for everybody
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kL) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    rd = rd + kStage == STAGES * kStage ? 0 : rd + kStage;
+    step(1, 0, true);
+    next_load();
+  }
+  wait_vmcnt<0>();
+
+  // a lane holds row m of C and, per accumulator, columns 4 q + {0..3} of a 16-column block
+  const int q = lane >> 4, r16 = lane & 15;
+  if (p.parts > 1) {
+    float* const P = p.part_ws + (int64_t)part * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+      const int m = m0 + wm + i * 16 + r16;
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < kNI; ++j) {
+        const int n = n0 + wn + j * 16 + 4 * q;
+        if (n < p.N) *reinterpret_cast<f32x4*>(P + (int64_t)m * p.N + n) = acc[j][i];
+      }
+    }
+    return;
+  }
+  if constexpr (OUT >= 2) {
+    float* const Cf = reinterpret_cast<float*>(C);
+    const bool fast = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(Cf) & 15) == 0);
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+      const int m = m0 + wm + i * 16 + r16;
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < kNI; ++j) {
+        const int n = n0 + wn + j * 16 + 4 * q;
+        float* cp = Cf + (int64_t)m * p.ldc + n;
+        if (fast && n + 4 <= p.N) {
+          f32x4 v = acc[j][i];
+          if (OUT == 3) v += *reinterpret_cast<const f32x4*>(cp);
+          *reinterpret_cast<f32x4*>(cp) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < p.N) cp[e] = (OUT == 3 ? cp[e] : 0.f) + acc[j][i][e];
+        }
+      }
+    }
+  } else {
+    uint16_t* const Cb = reinterpret_cast<uint16_t*>(C);
+    const bool fast = (p.ldc % 8 == 0) && ((reinterpret_cast<uintptr_t>(Cb) & 15) == 0);
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+      const int m = m0 + wm + i * 16 + r16;
+#pragma unroll
+      for (int j = 0; j < kNI; j += 2) {
+        f32x4 a = acc[j][i], b = acc[j + 1][i];
+        if (OUT == 1 && m < M) {
+          const int na = n0 + wn + j * 16 + 4 * q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (na + e < p.N) a[e] += bf16_bits_to_f32(Cb[(int64_t)m * p.ldc + na + e]);
+            if (na + 16 + e < p.N) b[e] += bf16_bits_to_f32(Cb[(int64_t)m * p.ldc + na + 16 + e]);
+          }
+        }
+        // odd groups of 16 lanes of block j <-> even groups of block j + 1: 8 consecutive columns per lane
+        const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
+        const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
+        u32x4 v;
+        v.x = s0[0]; v.y = s1[0]; v.z = s0[1]; v.w = s1[1];
+        const int n = n0 + wn + (j + (q & 1)) * 16 + 4 * (q & 2);
+        if (m >= M) continue;
+        if (fast && n + 8 <= p.N) {
+          *reinterpret_cast<u32x4*>(&Cb[(int64_t)m * p.ldc + n]) = v;
+        } else {
+          const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (n + e < p.N) Cb[(int64_t)m * p.ldc + n + e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    }
+  }
+}
+
+}  // namespace tile
+}  // namespace spx

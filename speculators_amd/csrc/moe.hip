@@ -97,6 +97,124 @@ __global__ __launch_bounds__(256) void pair_dot_kernel(const uint16_t* __restric
   if (lane == 0) out[pair] = sum;
 }
 
+// ---------------------------------------------------------------- (token, slot) pairs sorted by expert
+// A stable counting sort in three launches.  A wave owns `per_wave` consecutive pairs (a multiple of 64): it counts
+// them per expert, the scan turns the counts into first positions (expert-major, waves in their order inside an
+// expert), and the wave walks its pairs again, 64 at a time, giving every pair the position of its expert's next free
+// row -- lanes of the same expert rank themselves by the ballots of the id's bits, lower lanes first, so the order
+// inside an expert is the order of the pairs.  Bound by latency.
+constexpr int kSortWaves = 4;         // waves per workgroup
+constexpr int kSortMaxExperts = 2048;  // LDS counters: kSortWaves * experts * 4 bytes
+
+__device__ __forceinline__ int sort_expert(const int64_t* __restrict__ idx, int64_t i, int experts) {
+  const int64_t e = idx[i];
+  return (int)(e < 0 ? 0 : e >= experts ? experts - 1 : e);
+}
+
+__global__ __launch_bounds__(64 * kSortWaves) void sort_count_kernel(const int64_t* __restrict__ idx, int64_t pairs,
+                                                                     int experts, int per_wave, int waves,
+                                                                     int32_t* __restrict__ counts) {
+  extern __shared__ int32_t cnt[];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wave = blockIdx.x * kSortWaves + w;
+  int32_t* const mine = cnt + w * experts;
+  for (int e = lane; e < experts; e += 64) mine[e] = 0;
+  __syncthreads();
+  const int64_t first = (int64_t)wave * per_wave, last = min(first + per_wave, pairs);
+  if (wave < waves)
+    for (int64_t i = first + lane; i < last; i += 64) atomicAdd(&mine[sort_expert(idx, i, experts)], 1);
+  __syncthreads();
+  if (wave < waves)
+    for (int e = lane; e < experts; e += 64) counts[(int64_t)wave * experts + e] = mine[e];
+}
+
+// counts[wave][e] -> first position of the wave's pairs of expert e; offsets[e] = first row of expert e
+__global__ __launch_bounds__(1024) void sort_scan_kernel(int32_t* __restrict__ counts, int experts, int waves,
+                                                         int32_t* __restrict__ offsets) {
+  __shared__ int32_t sums[1024];
+  const int t = threadIdx.x;
+  const int per = (experts + 1023) / 1024;  // experts a thread: one contiguous run
+  int total = 0;
+  for (int j = 0; j < per; ++j) {
+    const int e = t * per + j;
+    if (e >= experts) break;
+    int run = 0;
+    int w = 0;
+    for (; w + 8 <= waves; w += 8) {
+      int32_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = counts[(int64_t)(w + u) * experts + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) run += v[u];
+    }
+    for (; w < waves; ++w) run += counts[(int64_t)w * experts + e];
+    total += run;
+  }
+  sums[t] = total;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {
+    const int v = t >= d ? sums[t - d] : 0;
+    __syncthreads();
+    sums[t] += v;
+    __syncthreads();
+  }
+  int at = sums[t] - total;
+  for (int j = 0; j < per; ++j) {
+    const int e = t * per + j;
+    if (e >= experts) break;
+    offsets[e] = at;
+    int w = 0;
+    for (; w + 8 <= waves; w += 8) {
+      int32_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = counts[(int64_t)(w + u) * experts + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        counts[(int64_t)(w + u) * experts + e] = at;
+        at += v[u];
+      }
+    }
+    for (; w < waves; ++w) {
+      const int v = counts[(int64_t)w * experts + e];
+      counts[(int64_t)w * experts + e] = at;
+      at += v;
+    }
+  }
+  if (t == 1023) offsets[experts] = sums[1023];
+}
+
+__global__ __launch_bounds__(64 * kSortWaves) void sort_scatter_kernel(
+    const int64_t* __restrict__ idx, int64_t pairs, int experts, int bits, int k, int per_wave, int waves,
+    const int32_t* __restrict__ counts, int64_t* __restrict__ order, int32_t* __restrict__ src_row,
+    int32_t* __restrict__ pos) {
+  extern __shared__ int32_t cnt[];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wave = blockIdx.x * kSortWaves + w;
+  if (wave >= waves) return;  // (no barrier below: a wave touches its own counters only)
+  volatile int32_t* const mine = cnt + w * experts;
+  for (int e = lane; e < experts; e += 64) mine[e] = counts[(int64_t)wave * experts + e];
+  const int64_t first = (int64_t)wave * per_wave, last = min(first + per_wave, pairs);
+  for (int64_t i0 = first; i0 < last; i0 += 64) {
+    const int64_t i = i0 + lane;
+    const bool live = i < last;
+    const int e = live ? sort_expert(idx, i, experts) : 0;
+    uint64_t same = __ballot(live);
+    for (int b = 0; b < bits; ++b) {
+      const uint64_t bal = __ballot((e >> b) & 1);
+      same &= ((e >> b) & 1) ? bal : ~bal;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1));
+    int at = 0;
+    if (live) at = mine[e] + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (live && rank == 0) mine[e] = at + __popcll(same);
+    __builtin_amdgcn_wave_barrier();
+    if (live) {
+      order[at] = i;
+      src_row[at] = (int32_t)(i / k);
+      pos[i] = at;
+    }
+  }
+}
+
 }  // namespace moe
 }  // namespace spx
 
@@ -145,4 +263,43 @@ extern "C" int spx_moe_pair_dot(const void* a, int64_t ld_a, const void* sorted,
                      reinterpret_cast<const uint16_t*>(sorted), ld_sorted, pos, out, pairs, (int)k, sorted_rows,
                      (int)(H / 8));
   return check_launch(__func__);
+}
+
+static int sort_plan(int64_t pairs, int& per_wave) {
+  // about 128 waves at most: the scan reads one row of counts per wave
+  per_wave = 256;
+  while ((pairs + per_wave - 1) / per_wave > 128) per_wave *= 2;
+  return (int)((pairs + per_wave - 1) / per_wave);
+}
+
+extern "C" int64_t spx_moe_sort_workspace_bytes(int64_t pairs, int64_t experts) {
+  if (pairs <= 0 || experts <= 0) return 0;
+  int per_wave;
+  return (int64_t)sort_plan(pairs, per_wave) * experts * (int64_t)sizeof(int32_t);
+}
+
+extern "C" int spx_moe_sort_pairs(const int64_t* idx, int64_t tokens, int32_t k, int64_t experts, int64_t* order,
+                                  int32_t* src_row, int32_t* pos, int32_t* offsets, void* workspace,
+                                  int64_t workspace_bytes, void* stream) {
+  SPX_REQUIRE(tokens > 0 && k > 0, "tokens and k must be positive");
+  SPX_REQUIRE(tokens * k < (1ll << 31), "too many pairs");
+  SPX_REQUIRE(experts > 0 && experts <= spx::moe::kSortMaxExperts, "1 .. 2048 experts");
+  SPX_REQUIRE(idx && order && src_row && pos && offsets && workspace, "null buffer");
+  SPX_REQUIRE(((uintptr_t)workspace) % 4 == 0, "unaligned workspace");
+  const int64_t pairs = tokens * k;
+  SPX_REQUIRE(workspace_bytes >= spx_moe_sort_workspace_bytes(pairs, experts), "workspace too small");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  int per_wave;
+  const int waves = sort_plan(pairs, per_wave);
+  int32_t* const counts = reinterpret_cast<int32_t*>(workspace);
+  const dim3 grid((unsigned)((waves + spx::moe::kSortWaves - 1) / spx::moe::kSortWaves)),
+      block(64 * spx::moe::kSortWaves);
+  const int smem = spx::moe::kSortWaves * (int)experts * 4;
+  int bits = 0;
+  while ((1ll << bits) < experts) ++bits;
+  hipLaunchKernelGGL(spx::moe::sort_count_kernel, grid, block, smem, st, idx, pairs, (int)experts, per_wave, waves, counts);
+  hipLaunchKernelGGL(spx::moe::sort_scan_kernel, dim3(1), dim3(1024), 0, st, counts, (int)experts, waves, offsets);
+  hipLaunchKernelGGL(spx::moe::sort_scatter_kernel, grid, block, smem, st, idx, pairs, (int)experts, bits, (int)k,
+                     per_wave, waves, counts, order, src_row, pos);
+  return spx::check_launch(__func__);
 }

@@ -43,6 +43,31 @@ def gemm_nt_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor,
     return out
 
 
+def gemm_nn_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor,
+                    out: torch.Tensor | None = None) -> torch.Tensor:
+    """``out[r] = a[r] @ b[e]`` for the rows ``offsets[e] <= r < offsets[e + 1]``: ``a [rows, K]``
+    sorted by group, ``b [groups, K, N]`` -- the input gradient of ``gemm_nt_grouped`` against the same
+    weight stack as it lies."""
+    if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
+        raise _lib.SpxError("gemm_nn_grouped takes bf16 operands")
+    if a.dim() != 2 or b.dim() != 3 or a.shape[1] != b.shape[1] or not b.is_contiguous():
+        raise ValueError(f"shape mismatch: a {tuple(a.shape)} b {tuple(b.shape)} (b contiguous)")
+    groups, k, n = b.shape
+    if offsets.dtype != torch.int32 or offsets.numel() != groups + 1 or offsets.device != a.device:
+        raise ValueError("offsets must be an int32 [groups + 1] tensor on the operands' device")
+    if a.stride(1) != 1:
+        a = a.contiguous()
+    rows = a.shape[0]
+    if out is None:
+        out = torch.empty(rows, n, device=a.device, dtype=torch.bfloat16)
+    nbytes = int(_lib.load().spx_gemm_grouped_workspace_bytes(rows, groups))
+    ws = torch.empty(nbytes // 4, device=a.device, dtype=torch.int32)
+    _lib.call("spx_gemm_bf16_nn_grouped", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(1), b.stride(0),
+              _lib.ptr(out), out.stride(0), rows, n, k, _lib.ptr(offsets), groups, _lib.ptr(ws), nbytes,
+              _lib.stream_ptr(a.device))
+    return out
+
+
 def gemm_tn_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor, out: torch.Tensor,
                     accumulate: bool = False) -> torch.Tensor:
     """``out[e] (+)= a[rows of e].T @ b[rows of e]``: ``a [rows, M]``, ``b [rows, N]`` sorted by
@@ -133,12 +158,12 @@ class _ExpertStacks:
         self.off[u].copy_(offsets)
         self.live = True
 
-    def add_gradient(self, acc):
+    def add_gradient(self, acc, dtype=torch.float32):
         if not self.live:
             return acc
         fresh = acc is None
         if fresh:
-            acc = torch.empty(self.w_shape, device=self.x.device, dtype=torch.float32)
+            acc = torch.empty(self.w_shape, device=self.x.device, dtype=dtype)
         gemm_tn_grouped_multi(self.dy, self.x, self.off, acc, accumulate=not fresh)
         self.off.zero_()  # uses whose backward does not run next time contribute nothing
         self.live = False
@@ -188,28 +213,44 @@ def route(logits: torch.Tensor, top_k: int, renormalise: bool):
     return top.to(logits.dtype), idx
 
 
+SORT_MAX_EXPERTS = 2048  # of spx_moe_sort_pairs
+
+
 def sort_pairs(idx: torch.Tensor, num_experts: int):
     """The ``(token, slot)`` pairs of ``idx [T, k]`` sorted by expert (stable: token order inside an
     expert).  -> ``order`` (pair of every sorted row, int64), ``src_row`` (its token, int32),
     ``pos`` (sorted row of every pair, int32 ``[T, k]``), ``offsets`` (int32 ``[E + 1]``).  All on
     the device; nothing is read back."""
     t, k = idx.shape
+    dev = idx.device
+    pairs = t * k
+    idx = idx.to(torch.int64).contiguous()
+    order = torch.empty(pairs, device=dev, dtype=torch.int64)
+    ints = torch.empty(2 * pairs + num_experts + 1, device=dev, dtype=torch.int32)
+    src_row, pos, offsets = ints[:pairs], ints[pairs:2 * pairs], ints[2 * pairs:]
+    if idx.is_cuda and num_experts <= SORT_MAX_EXPERTS and pairs:
+        nbytes = int(_lib.load().spx_moe_sort_workspace_bytes(pairs, num_experts))
+        ws = torch.empty(nbytes // 4, device=dev, dtype=torch.int32)
+        _lib.call("spx_moe_sort_pairs", _lib.ptr(idx), t, k, num_experts, _lib.ptr(order), _lib.ptr(src_row),
+                  _lib.ptr(pos), _lib.ptr(offsets), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev))
+        return order, src_row, pos.view(t, k), offsets
+    # host tensors, and more experts than the kernel's counters hold in LDS
     flat = idx.reshape(-1)
     order = torch.argsort(flat, stable=True)
-    counts = torch.zeros(num_experts, device=idx.device, dtype=torch.int32)
+    counts = torch.zeros(num_experts, device=dev, dtype=torch.int32)
     counts.index_add_(0, flat, torch.ones_like(flat, dtype=torch.int32))
-    offsets = torch.zeros(num_experts + 1, device=idx.device, dtype=torch.int32)
+    offsets[0] = 0
     offsets[1:] = counts.cumsum(0)
-    src_row = (order // k).to(torch.int32)
-    pos = torch.empty(t * k, device=idx.device, dtype=torch.int32)
-    pos[order] = torch.arange(t * k, device=idx.device, dtype=torch.int32)
+    src_row.copy_(order // k)
+    pos[order] = torch.arange(pairs, device=dev, dtype=torch.int32)
     return order, src_row, pos.view(t, k), offsets
 
 
 class _ExpertsMLP(torch.autograd.Function):
     """``Qwen3NextExperts.forward``: ``out[t] = sum_j scores[t, j] * down_e(silu(gate_e x_t) * up_e x_t)``,
     ``e = idx[t, j]``, on expert-sorted rows.  The weight gradients of the uses of one forward add
-    up in one fp32 buffer per weight (``Staged.grad_buffer``), which the staging node hands to
+    up in one buffer per weight (``Staged.grad_buffer``: fp32, or bf16 for the only use of bf16
+    parameters), which the staging node hands to
     autograd once."""
 
     @staticmethod
@@ -217,6 +258,8 @@ class _ExpertsMLP(torch.autograd.Function):
         if x2.dtype != torch.bfloat16:
             raise _lib.SpxError("the HIP layer kernels take bf16 tensors")
         w_gu, w_dn = st_gu.w, st_dn.w  # [E, 2I, H], [E, H, I]
+        st_gu.applied += 1
+        st_dn.applied += 1
         e, i2, h = w_gu.shape
         inter = i2 // 2
         order, src_row, pos, off = sort_pairs(idx, e)
@@ -257,14 +300,14 @@ class _ExpertsMLP(torch.autograd.Function):
         want_gu, want_dn = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
         dys = gather_rows(dout, src_row, wts.reshape(-1)[order].contiguous(),
                           out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
-        dact = gemm_nt_grouped(dys, st_dn.wt, off)
+        dact = gemm_nn_grouped(dys, st_dn.w, off)
         dh = (stack_gu.dy_slot(use_gu) if stack_gu is not None and want_gu
               else torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16))
         _lib.call("spx_swiglu_rows_bwd", _lib.ptr(hid), i2, _lib.ptr(hid[:, inter:]), i2, _lib.ptr(dact), inter,
                   _lib.ptr(dh), i2, _lib.ptr(dh[:, inter:]), i2, rows, inter, st)
         dx = None
         if ctx.needs_input_grad[0]:
-            dx = combine_rows(gemm_nt_grouped(dh, st_gu.wt, off), pos, None)
+            dx = combine_rows(gemm_nn_grouped(dh, st_gu.w, off), pos, None)
         marks = []
         for need, staged, dy2, x2, stack, use in ((want_gu, st_gu, dh, xs, stack_gu, use_gu),
                                                  (want_dn, st_dn, dys, act, stack_dn, use_dn)):

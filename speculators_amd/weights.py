@@ -117,9 +117,9 @@ class Staged:
     is expected to run against it (the size of the input / output-gradient buffers)."""
 
     __slots__ = ("w", "token", "rows_of", "uses", "_wt", "_xs", "_fill", "_dys", "_live", "_extras",
-                 "_marked", "_acc", "aux", "_finishers", "_task")
+                 "_marked", "_acc", "aux", "_finishers", "_task", "applied", "bf16_params")
 
-    def __init__(self, w, rows_of, uses: int = 1):
+    def __init__(self, w, rows_of, uses: int = 1, bf16_params: bool = False):
         self.w = w
         self.token = None  # fp32 stand-in of w's shape that carries the gradient edge (trainable only)
         self.rows_of = rows_of
@@ -131,9 +131,11 @@ class Staged:
         self._live = []    # (first row, rows) of the uses whose backward has run
         self._extras = []  # (dy, x) of uses outside the buffers
         self._marked = False
-        self._acc = None   # fp32 gradient buffer of uses that add their gradient themselves
+        self._acc = None   # gradient buffer of uses that add their gradient themselves
+        self.applied = 0   # products of this forward whose gradient goes to that buffer
+        self.bf16_params = bf16_params  # the parameters are bf16: a gradient written once may be bf16 itself
         self.aux = None    # whatever a family of products keeps per staged weight (the expert stacks)
-        self._finishers = []  # callables acc -> acc that add deferred gradients when the node runs
+        self._finishers = []  # callables (acc, dtype of a fresh acc) -> acc that add deferred gradients at the end
         self._task = None     # the backward pass (autograd graph task) the recorded uses belong to
 
     @property
@@ -218,13 +220,17 @@ class Staged:
         return torch.zeros(1, device=self.w.device, dtype=torch.float32).expand(self.w.shape)
 
     def grad_buffer(self):
-        """``(buffer, holds)``: the fp32 buffer of ``w``'s shape that uses which compute their weight
+        """``(buffer, holds)``: the buffer of ``w``'s shape that uses which compute their weight
         gradient themselves (the grouped expert products) add it to, and whether an earlier use of
-        this backward has written it already (the first one overwrites)."""
+        this backward has written it already (the first one overwrites).  fp32 -- or bf16 when this is
+        the forward's only use and the parameters are bf16: the same fp32 accumulation and the same one
+        rounding as a cast of the fp32 buffer."""
         self._enter_pass()
         holds = self._acc is not None
         if not holds:
-            self._acc = torch.empty(self.w.shape, device=self.w.device, dtype=torch.float32)
+            once = self.bf16_params and self.applied == 1
+            self._acc = torch.empty(self.w.shape, device=self.w.device,
+                                    dtype=torch.bfloat16 if once else torch.float32)
         return self._acc, holds
 
     def finish(self, bf16_ok: bool = False):
@@ -251,8 +257,10 @@ class Staged:
             acc = wgrad_product(self._dys[r0:r0 + n], self._xs[r0:r0 + n], acc)
         for dy2, x2 in self._extras:
             acc = wgrad_product(dy2, x2, acc)
-        for add_deferred in self._finishers:
-            acc = add_deferred(acc)
+        last = len(self._finishers) - 1
+        for i, add_deferred in enumerate(self._finishers):
+            # (a gradient that is one product writes bf16 itself, as above)
+            acc = add_deferred(acc, torch.bfloat16 if bf16_ok and i == last else torch.float32)
         self._dys, self._live, self._extras, self._marked, self._acc = None, [], [], False, None
         return acc
 
@@ -352,7 +360,7 @@ class WeightStager:
                 raise _lib.SpxError("libspx_hip works on HIP device tensors only (got a CPU parameter)")
         rows_of = [p.shape[0] for p in params]
         if torch.is_grad_enabled() and any(p.requires_grad for p in params):
-            st = Staged(None, rows_of, self._uses)
+            st = Staged(None, rows_of, self._uses, all(p.dtype == torch.bfloat16 for p in params))
             st.w, st.token = _Stage.apply(st, *params)
         else:
             fkey = tuple((p.data_ptr(), p._version, p.dtype) for p in params)

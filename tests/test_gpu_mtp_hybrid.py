@@ -40,8 +40,52 @@ def test_grouped_nt_product(sizes, n, k):
         r0 += sz
 
 
+@pytest.mark.parametrize("sizes,n,k", [([5, 0, 300, 129, 1, 0, 77], 264, 136), ([512], 512, 64), ([0, 0, 3], 8, 8),
+                                       ([257, 255, 256, 700], 520, 1000), ([1800], 264, 72)])
+def test_grouped_nn_product(sizes, n, k):
+    """Rows sorted by group against weights stored [K, N]: both tile heights (up to and above 256 rows a group on
+    average), empty groups, ragged N and K; and the transposed-weight product gives the same rows."""
+    from speculators_amd.moe import gemm_nn_grouped, gemm_nt_grouped
+
+    g = torch.Generator().manual_seed(sum(sizes) + n)
+    rows = sum(sizes)
+    a = torch.randn(rows, k, generator=g).bfloat16()
+    b = torch.randn(len(sizes), k, n, generator=g).bfloat16()
+    off = _groups(sizes)
+    out = torch.full((rows + 3, n), 7.0, dtype=torch.bfloat16, device="cuda")
+    got = gemm_nn_grouped(a.cuda(), b.cuda(), off.cuda(), out=out[:rows])
+    other = gemm_nt_grouped(a.cuda(), b.transpose(1, 2).contiguous().cuda(), off.cuda())
+    assert (out[rows:] == 7).all()
+    r0 = 0
+    for e, sz in enumerate(sizes):
+        want = a[r0:r0 + sz].float() @ b[e].float()
+        for x in (got, other):
+            if sz:
+                err = (x[r0:r0 + sz].float().cpu() - want).abs().max().item()
+                assert err <= 2 ** -8 * want.abs().max().item() + 1e-3, (e, err)
+        r0 += sz
+
+
+@pytest.mark.parametrize("t,k,experts", [(1, 1, 1), (37, 3, 5), (256, 1, 2048), (4099, 10, 512), (6000, 8, 3), (9, 2, 2049)])
+def test_sort_pairs_is_stable_on_the_device(t, k, experts):
+    """One wave and many, wave shares that end inside a 64-pair step, few experts (long runs of one id) and the
+    largest count the kernel takes; one more goes the other way."""
+    from speculators_amd import moe
+
+    g = torch.Generator().manual_seed(t + k)
+    idx = torch.randint(0, experts, (t, k), generator=g)
+    order, src_row, pos, off = moe.sort_pairs(idx.cuda(), experts)
+    want = torch.argsort(idx.reshape(-1), stable=True)
+    assert torch.equal(order.cpu(), want)
+    assert torch.equal(src_row.cpu(), (want // k).int())
+    assert torch.equal(order.cpu()[pos.cpu().reshape(-1).long()], torch.arange(t * k))
+    counts = torch.bincount(idx.reshape(-1), minlength=experts)
+    assert off[0] == 0 and torch.equal(off.cpu()[1:], counts.cumsum(0).int())
+
+
 @pytest.mark.parametrize("sizes,m,n", [([5, 0, 300, 64, 1, 0, 77], 264, 136), ([0, 0, 3], 8, 8),
-                                       ([130, 255, 70], 512, 520)])
+                                       ([130, 255, 70], 512, 520),
+                                       ([2100], 264, 72)])
 @pytest.mark.parametrize("fp32", [False, True])
 def test_grouped_tn_product(sizes, m, n, fp32):
     """Per-group weight gradients dY_e^T X_e: an empty group gets zeros, or is left alone when the
