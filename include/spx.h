@@ -200,6 +200,23 @@ int spx_label_ce_bwd_packed(const void* logits, int64_t ld_logits, const int64_t
                             const int32_t* row_map, void* dlogits, int64_t ld_out,
                             void* stream);
 
+/* Host side of the batch producer: fills a pinned staging buffer and uploads it.  Every segment is `bytes` bytes to
+ * `dst` (host), read from file descriptor `fd` at `offset` (fd >= 0) or copied from `src` (fd < 0; src == dst: already
+ * there).  Segments with dst inside [host, host + bytes) must come in ascending order and cover what is to be uploaded:
+ * the buffer goes to `device` on `stream` piece by piece as the pieces land (`threads` of the caller's process copy
+ * them; small batches are copied by the calling thread).  Returns when every segment has been copied and every upload
+ * enqueued; 1 if a file cannot be read.  Replaces the per-sample loads and the .to(device) of train/data.py:293-393
+ * and train/trainer.py:452-457. */
+typedef struct spx_stage_segment {
+  const void* src;  /* host */
+  void* dst;        /* host */
+  int64_t offset;
+  int64_t bytes;
+  int32_t fd;
+} spx_stage_segment;
+int spx_stage_upload(const spx_stage_segment* segments, int64_t n_segments, const void* host, void* device,
+                     int64_t bytes, int32_t threads, void* stream);
+
 /* Batch layout producer: packs `n_docs` samples, staged back to back in the layout
  * of the hidden-state files (`src_hs [n_src_rows, layers + 1, hidden]`, bf16 or fp32,
  * with `src_ids [n_src_rows]` int64 and `src_mask [n_src_rows]` of `mask_elem`-byte

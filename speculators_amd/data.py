@@ -5,8 +5,8 @@ The reference builds its batch on the host (train/data.py:293-303 splits the lay
 file, models/eagle3/data.py:8-44 shifts tokens against hidden states, ``CollateFn``
 train/data.py:323-393 packs samples into ``[1, max_len, ...]`` with ``document_ids``)
 and then copies six tensors to the device (train/trainer.py:452-457).  Here the raw
-file tensors are read straight into pinned host buffers, uploaded once on a side
-stream, and ``spx_pack_batch`` produces every tensor of the batch on the device: the
+file tensors are read straight into pinned host buffers by several threads, every piece
+uploaded on a side stream as soon as it is there (``spx_stage_upload``), and ``spx_pack_batch`` produces every tensor of the batch on the device: the
 layer split, the shift, the bf16 cast, the truncation at ``max_len``, the zero padding,
 ``position_ids`` and ``document_ids``.  ``PackedBatchLoader`` stages batch i+1 on a
 worker thread while the model runs on batch i.
@@ -29,6 +29,7 @@ Every layout also returns ``input_ids``, ``loss_mask``, ``position_ids`` and
 from __future__ import annotations
 
 import json
+import os
 import queue
 import struct
 import threading
@@ -92,6 +93,10 @@ class HiddenStatesFile:
         self.seq_len, self.layers_plus_one, self.hidden_size = hs.shape
         self.dtype = hs.dtype
 
+    def data_offset(self, name: str) -> int:
+        """Where the bytes of a tensor start in the file."""
+        return self._data_offset + self.entries[name].begin
+
     def read_into(self, name: str, dst: torch.Tensor) -> None:
         """Fill ``dst`` (contiguous CPU tensor of the entry's dtype and element count)."""
         e = self.entries[name]
@@ -138,21 +143,29 @@ def plan_rows(lengths, max_len: int, shift: int):
 
 
 class _Slot:
-    """Pinned staging + device staging for one batch in flight."""
+    """Pinned staging + device staging for one batch in flight: the hidden states, and beside them one
+    small buffer that holds the row plan, the token ids and the loss mask (one upload)."""
 
     def __init__(self, rows: int, layers_plus_one: int, hidden: int, src_dtype, mask_dtype,
                  max_docs: int, device):
         self.hs = torch.empty(rows, layers_plus_one, hidden, dtype=src_dtype, pin_memory=True)
-        self.ids = torch.empty(rows, dtype=torch.int64, pin_memory=True)
-        self.mask = torch.empty(rows, dtype=mask_dtype, pin_memory=True)
-        self.plan = torch.zeros(2, max_docs + 1, dtype=torch.int64, pin_memory=True)
         self.d_hs = torch.empty_like(self.hs, device=device)
-        self.d_ids = torch.empty_like(self.ids, device=device)
-        self.d_mask = torch.empty_like(self.mask, device=device)
-        self.d_plan = torch.empty_like(self.plan, device=device)
+        plan_bytes, id_bytes = 16 * (max_docs + 1), 8 * rows
+        mask_size = torch.empty(0, dtype=mask_dtype).element_size()
+        self.small = torch.empty(plan_bytes + id_bytes + mask_size * rows, dtype=torch.uint8, pin_memory=True)
+        self.small[:plan_bytes].zero_()
+        self.d_small = torch.empty_like(self.small, device=device)
+
+        def views(buf):
+            ids_end = plan_bytes + id_bytes
+            return (buf[:plan_bytes].view(torch.int64).view(2, max_docs + 1),
+                    buf[plan_bytes:ids_end].view(torch.int64), buf[ids_end:].view(mask_dtype))
+
+        self.plan, self.ids, self.mask = views(self.small)
+        self.d_plan, self.d_ids, self.d_mask = views(self.d_small)
         self.rows = 0
         self.n_docs = 1
-        self.done = None  # event: the pack kernel of the last use has finished
+        self.done = torch.cuda.Event()  # the uploads (then the pack kernel) of the last use have finished
         self.free = threading.Event()  # set once the last use has been handed to the device
         self.free.set()
 
@@ -191,6 +204,9 @@ class BatchPacker:
         self._next = 0
         self._abort = False
         self.stream = torch.cuda.Stream(device=self.device)
+        # threads that copy one batch into pinned memory (half of what the process may use, at most 8:
+        # the copies of eight outrun the upload)
+        self.copy_threads = max(1, min(8, len(os.sched_getaffinity(0)) // 2))
 
     def _slot(self) -> _Slot:
         i = self._next
@@ -204,16 +220,17 @@ class BatchPacker:
             if self._abort:
                 raise RuntimeError("batch staging abandoned")
         slot.free.clear()
-        if slot.done is not None:
-            slot.done.synchronize()  # its previous upload and pack have drained
+        slot.done.synchronize()  # its previous upload and pack have drained
         return slot
 
     def stage(self, samples) -> _Slot:
-        """Host part: copy / read the samples into a pinned slot and write the row plan."""
+        """Host part: copy / read the samples into a pinned slot, write the row plan and enqueue the
+        uploads on the packer's side stream (a piece goes to the device as soon as it is staged)."""
         slot = self._slot()
         try:
             self._fill(slot, samples)
         except BaseException:
+            self.stream.synchronize()  # what was enqueued before the error reads the slot
             slot.free.set()  # a rejected batch leaves the slot reusable
             raise
         return slot
@@ -221,6 +238,7 @@ class BatchPacker:
     def _fill(self, slot: _Slot, samples) -> None:
         lengths, at = [], 0
         room = self.max_len  # packed rows still free
+        jobs = []  # (sample, first staged row, rows) of what is staged
         for s in samples:
             if s is None:
                 continue
@@ -244,50 +262,89 @@ class BatchPacker:
                 raise ValueError(f"batch needs more than max_source_rows={self.max_source_rows} "
                                  "staged rows")
             if keep:
-                if is_file and keep == seq:
-                    hs.read_into("hidden_states", slot.hs[at:at + seq])
-                    hs.read_into("token_ids", slot.ids[at:at + seq])
-                else:
-                    loaded = hs.load() if is_file else {"hidden_states": hs, "token_ids": s["token_ids"]}
-                    slot.hs[at:at + keep].copy_(loaded["hidden_states"][:keep])
-                    slot.ids[at:at + keep].copy_(loaded["token_ids"][:keep])
-                slot.mask[at:at + keep].copy_(s["loss_mask"][:keep])
+                jobs.append((s, at, keep))
             lengths.append(keep)
             at += keep
             room -= max(keep - self.shift, 0)
         if not lengths:
             lengths = [0]
         src, out = plan_rows(lengths, self.max_len, self.shift)
-        slot.plan[0, :len(src)] = torch.tensor(src, dtype=torch.int64)
-        slot.plan[1, :len(out)] = torch.tensor(out, dtype=torch.int64)
+        slot.plan[:, :len(src)] = torch.tensor([src, out], dtype=torch.int64)
         slot.rows, slot.n_docs = at, len(lengths)
+        self._copy_and_upload(slot, jobs)
+
+    def _copy_and_upload(self, slot: _Slot, jobs) -> None:
+        with torch.cuda.device(self.device):
+            for i in range(0, len(jobs), 128):  # (a file stays open while its group is copied)
+                self._copy_group(slot, jobs[i:i + 128])
+            with torch.cuda.stream(self.stream):
+                if slot.small.numel() <= 1 << 20:
+                    slot.d_small.copy_(slot.small, non_blocking=True)
+                else:
+                    n = slot.rows
+                    slot.d_plan.copy_(slot.plan, non_blocking=True)
+                    slot.d_ids[:n].copy_(slot.ids[:n], non_blocking=True)
+                    slot.d_mask[:n].copy_(slot.mask[:n], non_blocking=True)
+                slot.done.record(self.stream)
+
+    def _copy_group(self, slot: _Slot, jobs) -> None:
+        row_bytes = (self.layers + 1) * self.hidden_size * slot.hs.element_size()
+        hs0, ids0 = slot.hs.data_ptr(), slot.ids.data_ptr()
+        ids_seg, hs_seg, fds = [], [], []
+        try:
+            for s, at, keep in jobs:
+                hs = s["hidden_states"]
+                slot.mask[at:at + keep].copy_(s["loss_mask"][:keep])
+                dst, n = hs0 + at * row_bytes, keep * row_bytes
+                if isinstance(hs, HiddenStatesFile):
+                    fd = os.open(hs.path, os.O_RDONLY)
+                    fds.append(fd)
+                    hs_seg.append((None, dst, hs.data_offset("hidden_states"), n, fd))
+                    if hs.entries["token_ids"].dtype == torch.int64:
+                        ids_seg.append((None, ids0 + 8 * at, hs.data_offset("token_ids"), 8 * keep, fd))
+                    else:
+                        ids = torch.empty(hs.seq_len, dtype=hs.entries["token_ids"].dtype)
+                        hs.read_into("token_ids", ids)
+                        slot.ids[at:at + keep].copy_(ids[:keep])
+                    continue
+                slot.ids[at:at + keep].copy_(s["token_ids"][:keep])
+                if hs.device.type == "cpu" and hs[:keep].is_contiguous():
+                    hs_seg.append((hs.data_ptr(), dst, 0, n, -1))
+                else:
+                    slot.hs[at:at + keep].copy_(hs[:keep])
+                    hs_seg.append((dst, dst, 0, n, -1))
+            segments = ids_seg + hs_seg
+            first = jobs[0][1] * row_bytes
+            nbytes = (jobs[-1][1] + jobs[-1][2]) * row_bytes - first
+            try:
+                _lib.call("spx_stage_upload", (_lib.StageSegment * len(segments))(*segments), len(segments),
+                          hs0 + first, _lib.ptr(slot.d_hs) + first, nbytes, self.copy_threads,
+                          self.stream.cuda_stream)
+            except _lib.SpxError as exc:
+                raise OSError(str(exc)) if fds else exc
+        finally:
+            for fd in fds:
+                os.close(fd)
 
     def pack(self, slot: _Slot) -> dict:
-        """Device part: one upload per staged tensor and one kernel, on the packer's side
-        stream; the returned tensors are ordered after them on the current stream."""
+        """Device part: one kernel on the packer's side stream, behind the slot's uploads; the returned
+        tensors are ordered after it on the current stream."""
         t, h, dev = self.max_len, self.hidden_size, self.device
         consumer = torch.cuda.current_stream(dev)
         with torch.cuda.stream(self.stream):
             n = slot.rows
-            if n:
-                slot.d_hs[:n].copy_(slot.hs[:n], non_blocking=True)
-                slot.d_ids[:n].copy_(slot.ids[:n], non_blocking=True)
-                slot.d_mask[:n].copy_(slot.mask[:n], non_blocking=True)
-            slot.d_plan.copy_(slot.plan, non_blocking=True)
             aux = (torch.empty(1, t, self.layers * h, device=dev, dtype=torch.bfloat16)
                    if self.has_aux else None)
             last = torch.empty(1, t, h, device=dev, dtype=torch.bfloat16)
-            ids = torch.empty(1, t, device=dev, dtype=torch.int64)
+            ints = torch.empty(3, 1, t, device=dev, dtype=torch.int64)
+            ids, pos, doc = ints[0], ints[1], ints[2]
             mask = torch.empty(1, t, device=dev, dtype=self.mask_dtype)
-            pos = torch.empty(1, t, device=dev, dtype=torch.int64)
-            doc = torch.empty(1, t, device=dev, dtype=torch.int64)
             _lib.call("spx_pack_batch", _lib.ptr(slot.d_hs), _lib.dtype_code(slot.d_hs), n,
                       self.layers, h, _lib.ptr(slot.d_ids), _lib.ptr(slot.d_mask),
                       slot.d_mask.element_size(), None, _lib.ptr(slot.d_plan[0]),
                       _lib.ptr(slot.d_plan[1]), slot.n_docs, t, self.shift, _lib.ptr(aux),
                       _lib.ptr(last), _lib.ptr(ids), _lib.ptr(mask), _lib.ptr(pos), _lib.ptr(doc),
                       self.stream.cuda_stream)
-            slot.done = torch.cuda.Event()
             slot.done.record(self.stream)
         slot.free.set()
         consumer.wait_event(slot.done)
@@ -295,7 +352,7 @@ class BatchPacker:
         if self.has_aux:
             batch["hidden_states"] = aux
         batch[self.last_key] = last
-        for v in batch.values():
+        for v in (ints, mask, last) + ((aux,) if self.has_aux else ()):
             v.record_stream(consumer)  # allocated on the side stream, consumed on this one
         return batch
 

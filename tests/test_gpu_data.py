@@ -142,6 +142,34 @@ def test_loader_over_hidden_state_files(tmp_path, layout):
     assert seen == len(batches)
 
 
+def test_pack_large_batch_from_files_and_memory(tmp_path):
+    """A batch above the size from which several threads stage it (pieces and uploads that end inside a document,
+    a document cut at the row's end, files and host tensors mixed, more documents than files open at a time), and a
+    file that ends early."""
+    from speculators_amd.data import BatchPacker, HiddenStatesFile
+
+    g = torch.Generator().manual_seed(2)
+    hidden, layers, max_len = 1024, 3, 3000
+    raws = [_raw(n, layers, hidden, g, torch.bfloat16) for n in [1, 900, 37, 1400] + [3] * 140 + [900]]
+    samples = []
+    for i, r in enumerate(raws):
+        if i % 2:
+            save_file({"hidden_states": r["hidden_states"], "token_ids": r["token_ids"]}, tmp_path / f"{i}.safetensors")
+            samples.append({"hidden_states": HiddenStatesFile(tmp_path / f"{i}.safetensors"),
+                            "loss_mask": r["loss_mask"]})
+        else:
+            samples.append(r)
+    packer = BatchPacker(max_len, hidden, layers, max_docs=256)
+    want = _want(raws, max_len, hidden, layers, "eagle3")
+    for _ in range(3):
+        _check(packer(samples), want)
+    path = tmp_path / "3.safetensors"
+    path.write_bytes(path.read_bytes()[:-1000])
+    with pytest.raises(OSError, match="ended before"):
+        packer(samples)
+    _check(packer([raws[1]]), _want([raws[1]], max_len, hidden, layers, "eagle3"))
+
+
 def test_loader_hands_worker_errors_to_the_caller(tmp_path):
     from speculators_amd.data import BatchPacker, PackedBatchLoader
 
