@@ -554,6 +554,21 @@ int spx_gemm_bf16_nt(const void* a, int64_t lda, const void* b, int64_t ldb,
                      void* c, int64_t ldc, int64_t M, int64_t N, int64_t K,
                      void* stream);
 
+/* The product on whichever kernel is predicted to be fastest for its size: form 0 c = a * b^T (b [N, K]), form 1
+ * c = a * b (b [K, N], row stride ldb; N a multiple of 8): the input gradient of a Linear on its weight as it lies.
+ * Products of few 256 x 256 tiles get smaller tiles or a contraction in parts (fp32 partials in the workspace, added
+ * in a fixed order, one rounding), the others run as spx_gemm_bf16_nt_tail does.  max_parts (1 .. 8) bounds the parts
+ * of that form's last round; 1: no contraction is ever cut.  m_live (device, may be NULL): the rows that count, as for
+ * spx_gemm_bf16_nt_rows.  workspace: spx_gemm_auto_workspace_bytes() bytes, 16-byte aligned (may be NULL when that is
+ * 0; a NULL workspace otherwise means no cut).  spx_gemm_auto_us: the predicted time in microseconds;
+ * spx_gemm_auto_tile: 0 when the product runs on the 256 x 256 kernel of spx_gemm_bf16_nt. */
+int64_t spx_gemm_auto_workspace_bytes(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts);
+float spx_gemm_auto_us(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts);
+int spx_gemm_auto_tile(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts);
+int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                       int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live,
+                       int32_t max_parts, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* spx_gemm_bf16_nt for products whose number of 256 x 256 output tiles leaves the last round of
  * workgroups mostly empty (384 tiles on 256 compute units: the second round is half empty and
  * takes as long as a full one).  The tiles of that last round -- when they are at most half a

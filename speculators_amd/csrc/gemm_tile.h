@@ -1,5 +1,11 @@
-// Small-tile bf16 GEMM kernels for gfx950 (NT, NN and TN forms, plain, cut along the contraction, grouped).
-// Instantiated and launched by gemm_tile.hip.
+// bf16 GEMM kernels for gfx950 on smaller tiles than those of gemm_bf16.hip (NT, NN and TN forms, plain, cut along
+// the contraction, grouped).  Instantiated, chosen and launched by gemm_tile.hip.
+//
+// Direct global -> LDS loads, STAGES slabs of 64 contraction indices deep, v_mfma_f32_16x16x32_bf16, operand
+// fragments double buffered in registers, the LDS reads of the next K step and the loads of the next free slab issued
+// between the products, one barrier per slab.  What bounds them is the way from L2 into LDS: 83 GB/s per compute unit
+// (21 TB/s over the chip; a kernel that only loads reaches 25) whatever the tile -- a slab of 128 x 128 takes 0.38 us
+// where its products need 0.26 -- so a larger tile is faster per multiply-add as long as every compute unit has one.
 #pragma once
 
 #include "spx_common.h"
@@ -118,6 +124,7 @@ struct Params {
   float* part_ws;               // [parts][M][N]
   const int32_t* tile_tab;      // grouped NT / NN: (group, first row) per tile row, see gemm_group_tiles_kernel
   const int32_t* group_off;     // grouped: group boundaries
+  const int32_t* m_live;        // how many leading rows of A count (device; null: all M)
   int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)
 };
 
@@ -138,11 +145,16 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   const uint16_t *A = p.A, *B = p.B;
   void* C = p.C;
   int tiles_m = p.tiles_m;
+  if (!AT && p.m_live) {  // the tile grid shrinks to the rows that count
+    M = min(M, max(*p.m_live, 0));
+    tiles_m = (M + TM - 1) / TM;
+  }
   if (!AT && p.tile_tab) tiles_m = min(p.tile_tab[0], tiles_m);
   const int n_tiles = tiles_m * p.tiles_n, n_wg = n_tiles * p.parts;
   if ((int)blockIdx.x >= n_wg) return;
-  // one contiguous run of tiles per XCD (workgroups go to the eight XCDs round robin), all parts of a tile in it:
-  // an XCD's tiles share their operand bands in its L2
+  // one contiguous run of workgroups per XCD (they go to the eight XCDs round robin), tiles in it first, then parts:
+  // an XCD's tiles share their operand bands in its L2, and with eight parts or more an XCD reads only its part of
+  // the contraction (12 % at 512 x 2048 x 8192 in 8 parts against all parts of a tile in one XCD)
   int pid;
   {
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, base = n_wg >> 3, rem = n_wg & 7;

@@ -8,6 +8,8 @@
 //   input gradient   595 us + 786 us to transpose the weights -> 459 us on the weights as they lie (NN form)
 //   weight gradient  bf16, 4 waves 760 us -> 8 waves 698 us (1067 us with the fp32 result it replaces)
 
+#include <algorithm>
+
 #include "gemm_tile.h"
 #include "gemm_tile_api.h"
 #include "../../include/spx.h"
@@ -126,6 +128,130 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
   }
 }
 
+// ------------------------------------------------------------------------------------------ plain products
+// C[m, n .. n + 7] = the sum of the parts of a product whose contraction was cut, in their order, fp32, one rounding
+__global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ C,
+                                                           int64_t ldc, int M_host, int N, int parts,
+                                                           const int32_t* __restrict__ m_live) {
+  const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
+  const int n8 = N / 8;
+  const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (item >= (int64_t)M * n8) return;
+  const int m = (int)(item / n8), n = (int)(item % n8) * 8;
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+  for (int p = 0; p < parts; ++p) {
+    const float* src = ws + ((int64_t)p * M_host + m) * N + n;
+    lo += *reinterpret_cast<const f32x4*>(src);
+    hi += *reinterpret_cast<const f32x4*>(src + 4);
+  }
+  u32x4 v;
+  v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
+  v.z = pack_bf16x2(hi[0], hi[1]); v.w = pack_bf16x2(hi[2], hi[3]);
+  *reinterpret_cast<u32x4*>(C + (int64_t)m * ldc + n) = v;
+}
+
+// The tile a product gets.  Every candidate's time is predicted and the shortest taken:
+//   rounds of workgroups x (slabs of a part x (s0 + s1 x filled share of the chip) + b)  [us], plus for a contraction
+//   in parts the pass that adds them, 4.1 + 1.03 per million fp32 partials.
+// s0, s1, b fitted to 180 products (M 256 .. 4096, the projections and heads of the 1B, 8B and 70B drafts and their
+// input gradients, 14 configurations each; 5 - 15 % rms).  On those products the choice is within 1.2 % of the best
+// candidate in the geometric mean and 1.33 x the 256 x 256 kernel alone (512 x 6144 -> 2048: 45.4 -> 23 us; 360 live
+// rows x 32000 -> 2048: 177 -> 62; 2000 x 4096 -> 4096: 71 -> 57; 4096-row products keep the large tile).
+enum Tile { kBig = 0, k128x128, k256x128, k64x128, k256x256 };
+struct Config {
+  int tm, tn, per_cu;
+  float s0, s1, b;
+};
+constexpr Config kNT[] = {{256, 256, 1, 1.18f, 0.23f, 6.9f},   // kBig: gemm_bf16.hip, its last round cut (tail_plan)
+                          {128, 128, 1, 0.35f, 0.14f, 4.1f},
+                          {256, 128, 1, 0.52f, 0.25f, 5.3f},
+                          {64, 128, 2, 0.18f, 0.42f, 3.0f}};
+constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (no 4-wave kernel of this form)
+                          {128, 128, 1, 0.43f, 0.125f, 0.6f},
+                          {256, 128, 1, 0.59f, 0.22f, 3.9f},
+                          {64, 128, 2, 0.25f, 0.48f, 0.f},
+                          {256, 256, 1, 1.13f, 0.33f, 4.0f}};
+constexpr int kCus = 256, kMinSlabs = 6, kMaxParts = 12, kSplitFrom = 32;  // (no cut below 32 slabs)
+
+struct Choice {
+  int tile, parts;
+  float us;
+};
+
+static float predict(const Config& c, int64_t tiles, int slabs) {
+  const int64_t cap = (int64_t)kCus * c.per_cu, full = tiles / cap, rem = tiles % cap;
+  float t = full * ((c.s0 + c.s1) * slabs + c.b);
+  if (rem) t += (c.s0 + c.s1 * (float)rem / (float)cap) * slabs + c.b;
+  return t;
+}
+
+static float reduce_us(int64_t elements) { return 4.1f + 1.03e-6f * (float)elements; }
+
+static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, bool can_split) {
+  const int slabs = (int)((K + kTK - 1) / kTK);
+  const bool nn = form == 1;
+  const Config* const table = nn ? kNN : kNT;
+  Choice best{kBig, 1, 1e30f};
+  if (!nn) {
+    const Config& c = table[kBig];
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), rem = tiles % kCus;
+    int64_t cut = 0;
+    int tp = 1;
+    if (max_parts > 1 && rem && rem * 2 <= kCus) {
+      tp = (int)std::min<int64_t>(kCus / rem, max_parts);
+      while (tp > 1 && slabs / tp < 16) --tp;
+      cut = tp > 1 ? rem : 0;
+    }
+    best.us = predict(c, tiles - cut, slabs);
+    if (cut) best.us += predict(c, cut * tp, (slabs + tp - 1) / tp) + reduce_us(cut * tp * 65536);
+  }
+  for (int t = 1; t < (nn ? 5 : 4); ++t) {
+    const Config& c = table[t];
+    const int64_t tiles = ((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
+    const int64_t cap = (int64_t)kCus * c.per_cu;
+    for (int parts = 1; parts <= kMaxParts; ++parts) {
+      // a cut fills a round that is not full, and only that
+      if (parts > 1 && (!can_split || max_parts <= 1 || slabs < kSplitFrom || slabs / parts < kMinSlabs ||
+                        tiles * parts > cap))
+        break;
+      float us = predict(c, tiles * parts, (slabs + parts - 1) / parts);
+      if (parts > 1) us += reduce_us(parts * M * N);
+      if (us < best.us) best = Choice{t, parts, us};
+    }
+  }
+  return best;
+}
+
+static int dense_check(const char* fname, int form, const void* a, int64_t lda, const void* b, int64_t ldb,
+                       const void* c, int64_t ldc, int64_t M, int64_t N, int64_t K) {
+  SPX_REQ_FN(form == 0 || form == 1, "form must be 0 (a b^T) or 1 (a b)");
+  SPX_REQ_FN(M > 0 && N > 0 && K > 0, "M, N, K must be positive");
+  SPX_REQ_FN(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "dimension too large");
+  SPX_REQ_FN(a && b && c, "null buffer");
+  SPX_REQ_FN(K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0, "K, lda, ldb must be multiples of 8");
+  SPX_REQ_FN(lda >= K && ldb >= (form ? N : K) && ldc >= N, "leading dimension too small");
+  SPX_REQ_FN(((uintptr_t)a | (uintptr_t)b) % 16 == 0, "a and b must be 16-byte aligned");
+  SPX_REQ_FN((256 * lda + K) * 2 < 0x7ffffff0ll, "256 rows of a must span less than 2 GiB (32-bit offsets)");
+  if (form == 0)
+    SPX_REQ_FN((256 * ldb + K) * 2 < 0x7ffffff0ll, "256 rows of b must span less than 2 GiB (32-bit offsets)");
+  else
+    SPX_REQ_FN(N % 8 == 0 && (K + 4 * kTK) * ldb * 2 < 0x7ffffff0ll,
+               "N must be a multiple of 8 and b span less than 2 GiB (32-bit offsets)");
+  return SPX_OK;
+}
+
+template <bool BT>
+static int launch_dense(const char* fname, int tile, const Params& p, hipStream_t st) {
+  switch (tile) {
+    case k128x128: return launch<128, 128, 2, 4, 4, 2, false, BT, 0>(fname, p, 1, st);
+    case k256x128: return launch<256, 128, 4, 2, 3, 2, false, BT, 0>(fname, p, 1, st);
+    case k64x128: return launch<64, 128, 2, 2, 3, 2, false, BT, 0>(fname, p, 1, st);
+    default:
+      if constexpr (BT) return launch<256, 256, 2, 4, 2, 2, false, true, 0>(fname, p, 1, st);
+      return fail_arg(fname, "no such tile");
+  }
+}
+
 }  // namespace tile
 }  // namespace spx
 
@@ -157,5 +283,64 @@ extern "C" int spx_gemm_bf16_nn_grouped(const void* a, int64_t lda, const void* 
   // rows 833 / 729 us
   return tile::grouped_rows<true>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups,
                                   workspace, rows > 256 * groups, reinterpret_cast<hipStream_t>(stream));
+}
+
+// whether the contraction of a product may be cut: the partials are stored in groups of four columns
+static bool can_split(int64_t N) { return N % 8 == 0; }
+
+extern "C" int64_t spx_gemm_auto_workspace_bytes(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts) {
+  if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1) return 0;
+  const tile::Choice c = tile::choose(form, M, N, K, max_parts, can_split(N));
+  if (c.tile == tile::kBig) return max_parts > 1 ? spx_gemm_tail_workspace_bytes() : 0;
+  return c.parts > 1 ? (int64_t)c.parts * M * N * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" float spx_gemm_auto_us(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts) {
+  if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1) return 0.f;
+  return tile::choose(form, M, N, K, max_parts, can_split(N)).us;
+}
+
+extern "C" int spx_gemm_auto_tile(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts) {
+  if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1) return 0;
+  return tile::choose(form, M, N, K, max_parts, can_split(N)).tile;
+}
+
+extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                                  int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live,
+                                  int32_t max_parts, void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* fname = __func__;
+  SPX_REQ_FN(max_parts >= 1 && max_parts <= 8, "max_parts must be 1 .. 8");
+  if (int rc = tile::dense_check(fname, form, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
+  const bool vec = ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;  // (what the pass that adds the parts stores)
+  const tile::Choice ch = tile::choose(form, M, N, K, max_parts, can_split(N) && vec && workspace);
+  if (ch.tile == tile::kBig) {
+    if (m_live) return spx_gemm_bf16_nt_rows(a, lda, b, ldb, c, ldc, M, N, K, m_live, stream);
+    if (max_parts > 1 && workspace && workspace_bytes >= spx_gemm_tail_workspace_bytes())
+      return spx_gemm_bf16_nt_tail(a, lda, b, ldb, c, ldc, M, N, K, max_parts, workspace, workspace_bytes, stream);
+    return spx_gemm_bf16_nt(a, lda, b, ldb, c, ldc, M, N, K, stream);
+  }
+  SPX_REQ_FN(ch.parts == 1 || (workspace_bytes >= (int64_t)ch.parts * M * N * (int64_t)sizeof(float) &&
+                               ((uintptr_t)workspace) % 16 == 0),
+             "workspace too small or unaligned");
+  const tile::Config& cfg = (form ? tile::kNN : tile::kNT)[ch.tile];
+  tile::Params p{};
+  p.A = reinterpret_cast<const uint16_t*>(a);
+  p.B = reinterpret_cast<const uint16_t*>(b);
+  p.C = c;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.M = (int)M; p.N = (int)N; p.K = (int)K;
+  const int64_t tiles_m = (M + cfg.tm - 1) / cfg.tm, tiles_n = (N + cfg.tn - 1) / cfg.tn;
+  SPX_REQ_FN(tiles_m * tiles_n * ch.parts < (1ll << 31), "too many tiles");
+  p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n; p.parts = ch.parts;
+  p.part_ws = reinterpret_cast<float*>(workspace);
+  p.m_live = m_live;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st))
+    return rc;
+  if (ch.parts == 1) return SPX_OK;
+  const int64_t items = M * (N / 8);
+  hipLaunchKernelGGL(tile::parts_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, p.part_ws,
+                     reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, ch.parts, m_live);
+  return check_launch(fname);
 }
 #undef SPX_REQ_FN

@@ -11,6 +11,7 @@ The models call the ``*_staged`` forms below with the compute weights of ``weigh
 
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -100,6 +101,73 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
             _lib.call("spx_gemm_bf16_nt_rows", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
                       _lib.ptr(out), out.stride(0), m, n, k, _lib.ptr(m_live), st)
     return out
+
+
+@functools.lru_cache(maxsize=4096)
+def _plan(form: int, m: int, n: int, k: int, parts: int):
+    """``(on the 256 x 256 kernel, workspace elements, predicted us)`` of ``spx_gemm_bf16_auto``."""
+    lib = _lib.load()
+    return (lib.spx_gemm_auto_tile(form, m, n, k, parts) == 0,
+            lib.spx_gemm_auto_workspace_bytes(form, m, n, k, parts) // 4,
+            lib.spx_gemm_auto_us(form, m, n, k, parts))
+
+
+def _auto(form: int, a, b, out, m: int, n: int, k: int, ws_numel: int, m_live=None):
+    if out is None:
+        out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
+    ws = _split_workspace(a.device, ws_numel) if ws_numel else None
+    _lib.call("spx_gemm_bf16_auto", form, _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0), _lib.ptr(out),
+              out.stride(0), m, n, k, _lib.ptr(m_live), TAIL_PARTS, _lib.ptr(ws), ws_numel * 4,
+              _lib.stream_ptr(a.device))
+    return out
+
+
+def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = None) -> torch.Tensor:
+    """``a[M, K] @ b[N, K].T`` (bf16) on the kernel its size asks for (``spx_gemm_bf16_auto``): products of
+    few 256 x 256 tiles on smaller tiles or with the contraction in parts, the others on ``gemm_nt``.
+    ``m_live`` as there (the 256 x 256 kernel then decides its parts from the row count)."""
+    m, k = a.shape
+    n = b.shape[0]
+    if m_live is not None and (m_live.dtype != torch.int32 or m_live.numel() != 1 or m_live.device != a.device):
+        raise ValueError("m_live must be a one-element int32 tensor on the operands' device")
+    if k == b.shape[1] and k % 8 == 0 and a.stride(1) == 1 and b.stride(1) == 1 and a.dtype == b.dtype == torch.bfloat16:
+        big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
+        if not big:
+            return _auto(0, a, b, None, m, n, k, ws_numel, m_live)
+    return gemm_nt(a, b, m_live=m_live, split=m_live is not None)
+
+
+def _nn_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether ``a[M, K] @ b[K, N]`` meets the alignment rules of the NN kernels."""
+    k, n = b.shape
+    return (a.dtype == b.dtype == torch.bfloat16 and k % 8 == 0 and n % 8 == 0 and a.stride(1) == 1
+            and b.stride(1) == 1 and a.stride(0) % 8 == 0 and b.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0
+            and b.data_ptr() % 16 == 0 and (k + 256) * b.stride(0) * 2 < _MAX_SPAN
+            and (256 * a.stride(0) + k) * 2 < _MAX_SPAN)
+
+
+def matmul_nn(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """``a[M, K] @ b[K, N]`` (bf16, ``_nn_fits``): the input gradient of a Linear on its weight as it
+    lies, no transposed copy of it."""
+    m, k = a.shape
+    n = b.shape[1]
+    return _auto(1, a, b, None, m, n, k, _plan(1, m, n, k, TAIL_PARTS)[1])
+
+
+# microseconds to transpose a million weight elements (spx_transpose_bf16: 4 bytes each at 3.8 TB/s)
+_TRANSPOSE_US = 1.05
+
+
+def input_gradient(dy2: torch.Tensor, staged) -> torch.Tensor:
+    """``dy2 @ staged.w``: on the weight as it lies (NN kernels) or on its transposed copy (NT kernels), whichever
+    is predicted to be faster -- the copy of a weight that trains is one per forward and is shared by the
+    weight's uses; that of a frozen weight is kept."""
+    if _nn_fits(dy2, staged.w):
+        m, (k, n) = dy2.shape[0], staged.w.shape
+        copy_us = 0.0 if staged.has_wt or not staged.trainable else (3.0 + _TRANSPOSE_US * 1e-6 * k * n) / staged.uses
+        if _plan(1, m, n, k, TAIL_PARTS)[2] <= _plan(0, m, n, k, TAIL_PARTS)[2] + copy_us:
+            return matmul_nn(dy2, staged.w)
+    return matmul_nt(dy2, staged.wt)
 
 
 def gemm_nt_stats(a: torch.Tensor, b: torch.Tensor, store: bool = True, want_argmax: bool = True,
@@ -210,7 +278,7 @@ class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, weight_t):
         x2 = x.reshape(-1, x.shape[-1])
-        y = gemm_nt(x2, weight)
+        y = matmul_nt(x2, weight)
         ctx.save_for_backward(x2, weight, weight_t)
         ctx.x_shape = x.shape
         return y.view(*x.shape[:-1], weight.shape[0])
@@ -221,8 +289,11 @@ class _Linear(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            wt = weight_t if weight_t is not None else weight.t().contiguous()
-            dx = gemm_nt(dy2, wt).view(ctx.x_shape)
+            if weight_t is None and _nn_fits(dy2, weight):
+                dx = matmul_nn(dy2, weight)
+            else:
+                dx = matmul_nt(dy2, weight_t if weight_t is not None else weight.t().contiguous())
+            dx = dx.view(ctx.x_shape)
         if ctx.needs_input_grad[1]:
             from .weights import wgrad_product
 
@@ -249,32 +320,34 @@ if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
     raise ValueError(f"SPX_DECODER_GEMM must be 'hipblaslt', 'spx' or 'mixed', got {DECODER_GEMM!r}")
 
 
-def _tail_cut_applies(m: int, n: int, k: int) -> bool:
-    """Whether ``gemm_nt`` cuts the last round of tiles of an ``[m, k] x [n, k]^T`` product (the rule of
-    ``spx_gemm_bf16_nt_tail``): the shapes on which a 256 x 256 tiling loses most to tile quantisation
-    and the cut wins it back (the merged q/k/v projection of the 8B shape: 384 tiles)."""
-    rem = (-(-m // 256) * -(-n // 256)) % _CUS
-    return TAIL_PARTS > 1 and 0 < rem <= _CUS // 2 and k >= 64 * 16 * 2 and (-(-m // 256) * -(-n // 256)) < 2 * _CUS
+def _own_forward(m: int, n: int, k: int) -> bool:
+    """Whether the forward product of a decoder projection runs on this library's kernels in "mixed": where the
+    smaller tiles fill the chip in one round (level with hipBLASLt or ahead: 0.65 - 1.0 of its time up to 1024 rows,
+    0.73 - 0.94 where the contraction is cut), and where the last round of the large tiles is cut along the
+    contraction (``spx_gemm_bf16_nt_tail``; the merged q/k/v projection of the 8B shape: 322 us, library 357)."""
+    big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
+    if not big:
+        return ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128
+    tiles = -(-m // 256) * -(-n // 256)
+    return TAIL_PARTS > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS
 
 
 def _project(x2: torch.Tensor, staged) -> torch.Tensor:
     """``x2 @ staged.w.T`` of a decoder-layer projection."""
     if DECODER_GEMM == "spx":
-        return gemm_nt(x2, staged.w)
-    if (DECODER_GEMM == "mixed" and x2.dtype == torch.bfloat16
-            and _tail_cut_applies(x2.shape[0], staged.w.shape[0], x2.shape[1])):
-        # (measured at [4096, 8192] x [6144, 8192]^T: 322 us here, 357 us on the library)
-        return gemm_nt(x2, staged.w)
+        return matmul_nt(x2, staged.w)
+    if DECODER_GEMM == "mixed" and x2.dtype == torch.bfloat16 and _own_forward(x2.shape[0], *staged.w.shape):
+        return matmul_nt(x2, staged.w)
     return torch.nn.functional.linear(x2, staged.w)
 
 
 def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
     """``dy2 @ staged.w``: the input gradient of a decoder-layer projection ("mixed": this one on the
-    library's kernel against the transposed copy, the forward product on hipBLASLt)."""
+    library's kernels, the forward product on hipBLASLt)."""
     # (the kernel contracts in chunks of 8: a projection a few columns wide -- a gate of width 1 --
     # stays with the library)
     if DECODER_GEMM != "hipblaslt" and dy2.shape[1] % 8 == 0 and dy2.stride(0) % 8 == 0 and dy2.stride(1) == 1:
-        return gemm_nt(dy2, staged.wt)
+        return input_gradient(dy2, staged)
     return torch.matmul(dy2, staged.w)
 
 
@@ -289,7 +362,7 @@ class _StagedLinear(torch.autograd.Function):
             raise _lib.SpxError("the HIP layer kernels take bf16 tensors")
         w = staged.w
         x2 = x.reshape(-1, x.shape[-1])
-        y = gemm_nt(x2, w) if hip else _project(x2, staged)
+        y = matmul_nt(x2, w) if hip else _project(x2, staged)
         ctx.save_for_backward(x2, w)
         ctx.staged, ctx.hip, ctx.x_shape = staged, hip, x.shape
         ctx.slot = staged.take(x2) if ctx.needs_input_grad[1] else -1
@@ -302,7 +375,7 @@ class _StagedLinear(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = (gemm_nt(dy2, ctx.staged.wt) if ctx.hip else _project_back(dy2, ctx.staged)).view(ctx.x_shape)
+            dx = (input_gradient(dy2, ctx.staged) if ctx.hip else _project_back(dy2, ctx.staged)).view(ctx.x_shape)
         if ctx.needs_input_grad[1]:
             dw = ctx.staged.defer(ctx.slot, dy2, x2)
         return dx, dw, None, None
@@ -312,7 +385,7 @@ def linear_staged(x: torch.Tensor, staged, hip: bool = False) -> torch.Tensor:
     """``x[..., K] @ staged.w[N, K].T``; see ``_StagedLinear``."""
     if not torch.is_grad_enabled() or not (x.requires_grad or staged.trainable):
         x2 = x.reshape(-1, x.shape[-1])
-        y = gemm_nt(x2, staged.w) if hip else _project(x2, staged)
+        y = matmul_nt(x2, staged.w) if hip else _project(x2, staged)
         return y.view(*x.shape[:-1], staged.w.shape[0])
     y = _StagedLinear.apply(x, staged.token, staged, hip)
     node = y.grad_fn

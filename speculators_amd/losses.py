@@ -281,9 +281,9 @@ class _HeadFusedLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, weight, weight_t, targets, op, known_lse_t, known_am_t, n_rows, step=None):
-        from .gemm import gemm_nt
+        from .gemm import matmul_nt
 
-        logits = gemm_nt(x2, weight)
+        logits = matmul_nt(x2, weight)
         known = (known_lse_t, known_am_t) if known_lse_t is not None else None
         ctx.op, ctx.total_rows = op, logits.shape[0]
         xs = logits[:n_rows]
@@ -302,14 +302,14 @@ class _HeadFusedLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_rows, _gd, _gt, _gl, _glogits):
-        from .gemm import gemm_nt
+        from .gemm import matmul_nt
 
         if grad_rows is None:
             return (None,) * 9
         if ctx.one_pass:
             packed, row_map, count, weight_t = ctx.saved_tensors
             g = grad_rows.reshape(-1).to(torch.float32).contiguous()
-            dx_packed = gemm_nt(packed, weight_t, m_live=count, split=True)
+            dx_packed = matmul_nt(packed, weight_t, m_live=count)
             return (_unpack_rows_scaled(dx_packed, row_map, g, ctx.total_rows), None, None, None, None, None,
                     None, None, None)
 
@@ -324,7 +324,7 @@ class _HeadFusedLoss(torch.autograd.Function):
             _lib.ptr(lse_d), _lib.ptr(lse_t), _lib.ptr(extra), _lib.ptr(am_t), _lib.ptr(g), None,
             _lib.ptr(row_map), _lib.ptr(packed), packed.stride(0), _lib.stream_ptr(x.device),
         )
-        dx_packed = gemm_nt(packed, weight_t, m_live=count, split=True)
+        dx_packed = matmul_nt(packed, weight_t, m_live=count)
         return (_unpack_rows(dx_packed, row_map, ctx.total_rows), None, None, None, None, None,
                 None, None, None)
 
@@ -504,7 +504,7 @@ class _HeadLabelCE(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, weight, weight_t, labels, ignore_index, epilogue_stats=False):
-        from .gemm import gemm_nt, gemm_nt_stats
+        from .gemm import gemm_nt_stats, matmul_nt
 
         if epilogue_stats:
             # the head product's epilogue leaves every row's log-sum-exp; the loss then reads one
@@ -517,7 +517,7 @@ class _HeadLabelCE(torch.autograd.Function):
                       vocab, _lib.dtype_code(logits), int(ignore_index), _lib.ptr(out[1]), _lib.ptr(out[0]),
                       _lib.stream_ptr(logits.device))
         else:
-            logits = gemm_nt(x2, weight)
+            logits = matmul_nt(x2, weight)
             rows, vocab = logits.shape
             out = torch.empty(2, rows, device=logits.device, dtype=torch.float32)
             _lib.call("spx_label_ce_fwd", _lib.ptr(logits), logits.stride(0), _lib.ptr(labels), rows,
@@ -531,7 +531,7 @@ class _HeadLabelCE(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_rows, _grad_logits):
-        from .gemm import gemm_nt
+        from .gemm import matmul_nt
 
         if grad_rows is None:
             return (None,) * 6
@@ -545,7 +545,7 @@ class _HeadLabelCE(torch.autograd.Function):
                   _lib.ptr(lse), _lib.ptr(g), rows, vocab, _lib.dtype_code(logits), ctx.ignore_index,
                   _lib.ptr(row_map), _lib.ptr(packed), packed.stride(0),
                   _lib.stream_ptr(logits.device))
-        dx_packed = gemm_nt(packed, weight_t, m_live=count, split=True)
+        dx_packed = matmul_nt(packed, weight_t, m_live=count)
         return _unpack_rows(dx_packed, row_map, rows), None, None, None, None, None
 
 

@@ -97,7 +97,7 @@ class VerifierHead:
         from . import gemm
 
         if self.logits is None:
-            self.logits = gemm.gemm_nt(self.x[0], self.weight).view(1, self.x.shape[1], self.weight.shape[0])
+            self.logits = gemm.matmul_nt(self.x[0], self.weight).view(1, self.x.shape[1], self.weight.shape[0])
         return self.logits
 
     def stats(self):

@@ -143,6 +143,10 @@ class Staged:
         return self.token is not None
 
     @property
+    def has_wt(self) -> bool:
+        return self._wt is not None
+
+    @property
     def wt(self) -> torch.Tensor:
         """``w.T`` contiguous (made on first use, kept with the staged weight)."""
         if self._wt is None:

@@ -481,3 +481,40 @@ def test_every_tile_of_a_ragged_tile_grid_is_computed_once(tiles):
     out32 = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
     gemm_tn(at, bt, out=out32)
     torch.testing.assert_close(out32, at.float().T @ bt.float(), rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 8), (63, 136, 72), (64, 128, 2048), (65, 256, 2056), (129, 1000, 2112), (257, 520, 6144), (360, 2048, 4000),
+    (512, 2048, 8192), (700, 3072, 4096), (1000, 1800, 2112), (1999, 2048, 2048), (2000, 4096, 512), (513, 4104, 136),
+])
+def test_product_on_the_tile_its_size_asks_for(form, m, n, k):
+    """``spx_gemm_bf16_auto`` in both forms at the edges of its tiles (64, 128, 256), with whole contractions and cut
+    ones, ragged in every direction: against the fp64 product, repeatable bit for bit, nothing written outside; with a
+    device-side row count the rows past it are neither read nor written and the others keep their bits."""
+    from speculators_amd import _lib, gemm
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    b = (torch.randn(*((n, k) if form == 0 else (k, n)), device="cuda", generator=g) / k ** 0.5).bfloat16()
+    want = a.double() @ (b.double().t() if form == 0 else b.double())
+    big, ws_numel, _ = gemm._plan(form, m, n, k, gemm.TAIL_PARTS)
+    ws = torch.empty(max(ws_numel, 1), device="cuda")
+    live = max(m - 70, 0)
+
+    def run(count, rows):
+        buf = torch.full((m + 2, n), 7.0, dtype=torch.bfloat16, device="cuda")
+        src = a.clone()
+        src[rows:] = float("nan")
+        _lib.call("spx_gemm_bf16_auto", form, _lib.ptr(src), k, _lib.ptr(b), b.stride(0), _lib.ptr(buf[1:]), n, m, n, k,
+                  _lib.ptr(count), gemm.TAIL_PARTS, _lib.ptr(ws) if ws_numel else None, ws_numel * 4,
+                  _lib.stream_ptr(a.device))
+        assert (buf[0] == 7).all() and (buf[1 + rows:] == 7).all()
+        return buf[1:1 + rows]
+
+    full = run(None, m)
+    assert (full.double() - want).abs().max().item() <= 1e-2 * want.abs().max().item()
+    assert torch.equal(full.view(torch.int16), run(None, m).view(torch.int16))
+    if not big:
+        some = run(torch.tensor([live], dtype=torch.int32, device="cuda"), live)
+        assert torch.equal(some.view(torch.int16), full[:live].view(torch.int16))
