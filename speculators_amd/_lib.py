@@ -151,11 +151,51 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The binding module (``csrc/binding.cpp``): every entry point as a function that takes integers,
+    floats, None and HIP tensors (where C takes a pointer) and raises ``SpxError`` on a failed status."""
+    global _native
+    if _native is None:
+        load()
+        if os.environ.get("SPX_LIB_PATH"):
+            _native = _CtypesCalls(_lib)  # another build of the library than the one beside this file
+        else:
+            try:
+                from . import _spx_native as mod
+            except ImportError as exc:
+                raise SpxError("speculators_amd/_spx_native.so is missing: build it with "
+                               "`make -C speculators_amd/csrc`; there is no fallback path") from exc
+            mod.set_error(SpxError)
+            _native = mod
+    return _native
+
+
+class _CtypesCalls:
+    """The functions of the binding module over a ``ctypes`` library."""
+
+    def __init__(self, lib):
+        self._lib = lib
+
+    def __getattr__(self, name):
+        fn = getattr(self._lib, name)
+        status = name not in RESTYPES and name not in ("spx_version", "spx_gemm_auto_tile")
+
+        def call_(*args):
+            rc = fn(*(ptr(a) if isinstance(a, torch.Tensor) else a for a in args))
+            if not status:
+                return rc
+            if rc != 0:
+                raise SpxError(f"{name} failed ({rc}): {self._lib.spx_last_error().decode()}")
+
+        setattr(self, name, call_)
+        return call_
+
+
 def call(name: str, *args) -> None:
-    lib = load()
-    rc = getattr(lib, name)(*args)
-    if rc != 0:
-        raise SpxError(f"{name} failed ({rc}): {lib.spx_last_error().decode()}")
+    getattr(_native or native(), name)(*args)
 
 
 def ptr(t: torch.Tensor | None):
@@ -168,7 +208,28 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream_ptr(device=None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of a device (an address; None for a host device, whose tensors no call takes)."""
+    if isinstance(device, torch.device):
+        if device.type != "cuda":
+            return None
+        index = device.index
+    else:
+        index = device
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+_zeros: dict = {}
+
+
+def zero(device, dtype=torch.float32) -> torch.Tensor:
+    """A one-element zero, kept per device: the memory behind empty gradient markers.  Never written."""
+    key = (device, dtype)
+    z = _zeros.get(key)
+    if z is None:
+        z = _zeros[key] = torch.zeros(1, device=device, dtype=dtype)
+    return z
 
 
 DTYPE_CODE = {torch.bfloat16: 0, torch.float32: 1}

@@ -23,7 +23,7 @@ ATTN_IMPL_DFLASH = "dflash_hip"
 
 
 def _workspace_bytes(t, hq, hkv, d, backward):
-    return int(_lib.load().spx_ttt_attn_workspace_bytes(t, hq, hkv, d, int(backward)))
+    return int(_lib.native().spx_ttt_attn_workspace_bytes(t, hq, hkv, d, int(backward)))
 
 
 @dataclass
@@ -56,8 +56,8 @@ def create_ttt_mask(document_ids: torch.Tensor, total_seq_len: int,
         doc = doc.to(torch.int64)
     doc = doc.contiguous()
     row_lo = torch.empty(total_seq_len, device=doc.device, dtype=torch.int32)
-    _lib.call("spx_ttt_row_lo", _lib.ptr(doc), _lib.kind_code(doc), total_seq_len,
-              int(sliding_window) if sliding_window else 0, _lib.ptr(row_lo),
+    _lib.call("spx_ttt_row_lo", doc, _lib.kind_code(doc), total_seq_len,
+              int(sliding_window) if sliding_window else 0, row_lo,
               _lib.stream_ptr(doc.device))
     return TTTMask(row_lo, total_seq_len, 0, sliding_window)
 
@@ -85,9 +85,9 @@ class _TTTAttention(torch.autograd.Function):
         out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
         lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_fwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(mask.row_lo), t, mask.ttt_step, hq, hkv, d,
-                  float(scaling), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws), ws.numel(),
+        _lib.call("spx_ttt_attn_fwd", q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), mask.row_lo, t, mask.ttt_step, hq, hkv, d,
+                  float(scaling), out, lse, ws, ws.numel(),
                   _lib.stream_ptr(dev))
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.mask, ctx.scaling = mask, float(scaling)
@@ -105,11 +105,11 @@ class _TTTAttention(torch.autograd.Function):
         dk = torch.empty_like(k)
         dv = torch.empty_like(v)
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_bwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(out), _lib.ptr(dout), _lib.ptr(lse),
-                  _lib.ptr(mask.row_lo), t, mask.ttt_step, hq, hkv, d, ctx.scaling,
-                  _lib.ptr(dq), dq.stride(1), _lib.ptr(dk), dk.stride(1), _lib.ptr(dv),
-                  dv.stride(1), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev))
+        _lib.call("spx_ttt_attn_bwd", q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), out, dout, lse,
+                  mask.row_lo, t, mask.ttt_step, hq, hkv, d, ctx.scaling,
+                  dq, dq.stride(1), dk, dk.stride(1), dv,
+                  dv.stride(1), ws, ws.numel(), _lib.stream_ptr(dev))
         return dq, dk, dv, None, None
 
 
@@ -165,9 +165,9 @@ class _TTTAttentionCached(torch.autograd.Function):
             out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
         lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_fwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(mask.row_lo), t, mask.ttt_step, hq, hkv, d,
-                  float(scaling), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws), ws.numel(),
+        _lib.call("spx_ttt_attn_fwd", q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), mask.row_lo, t, mask.ttt_step, hq, hkv, d,
+                  float(scaling), out, lse, ws, ws.numel(),
                   _lib.stream_ptr(dev))
         ctx.save_for_backward(q, out, lse)
         ctx.kv = (k, v)  # windows of the cache: later steps only write rows beyond them
@@ -201,11 +201,11 @@ class _TTTAttentionCached(torch.autograd.Function):
             if shared:
                 g.task, g.dk, g.dv = task, dk, dv
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call(entry, _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(out), _lib.ptr(dout), _lib.ptr(lse),
-                  _lib.ptr(mask.row_lo), t, mask.ttt_step, hq, hkv, d, ctx.scaling,
-                  _lib.ptr(dq), dq.stride(1), _lib.ptr(dk), dk.stride(1), _lib.ptr(dv),
-                  dv.stride(1), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev))
+        _lib.call(entry, q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), out, dout, lse,
+                  mask.row_lo, t, mask.ttt_step, hq, hkv, d, ctx.scaling,
+                  dq, dq.stride(1), dk, dk.stride(1), dv,
+                  dv.stride(1), ws, ws.numel(), _lib.stream_ptr(dev))
         if not shared:  # outside a backward pass of the engine: every step's window, to be summed by the caller
             dks = [dk[:, :, i * t:(i + 1) * t] for i in range(n)]
             dvs = [dv[:, :, i * t:(i + 1) * t] for i in range(n)]
@@ -318,9 +318,9 @@ class _SpanAttention(torch.autograd.Function):
         out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
         lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_span_attn_fwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1), _lib.ptr(v),
-                  v.stride(1), _lib.ptr(mask.row_lo), _lib.ptr(mask.row_hi), t, hq, hkv, d, float(scaling),
-                  _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev))
+        _lib.call("spx_span_attn_fwd", q, q.stride(1), k, k.stride(1), v,
+                  v.stride(1), mask.row_lo, mask.row_hi, t, hq, hkv, d, float(scaling),
+                  out, lse, ws, ws.numel(), _lib.stream_ptr(dev))
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.mask, ctx.scaling = mask, float(scaling)
         return out
@@ -335,10 +335,10 @@ class _SpanAttention(torch.autograd.Function):
         dout = dout.to(torch.bfloat16).contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call("spx_span_attn_bwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1), _lib.ptr(v),
-                  v.stride(1), _lib.ptr(out), _lib.ptr(dout), _lib.ptr(lse), _lib.ptr(mask.row_lo),
-                  _lib.ptr(mask.row_hi), t, hq, hkv, d, ctx.scaling, _lib.ptr(dq), dq.stride(1),
-                  _lib.ptr(dk), dk.stride(1), _lib.ptr(dv), dv.stride(1), _lib.ptr(ws), ws.numel(),
+        _lib.call("spx_span_attn_bwd", q, q.stride(1), k, k.stride(1), v,
+                  v.stride(1), out, dout, lse, mask.row_lo,
+                  mask.row_hi, t, hq, hkv, d, ctx.scaling, dq, dq.stride(1),
+                  dk, dk.stride(1), dv, dv.stride(1), ws, ws.numel(),
                   _lib.stream_ptr(dev))
         return dq, dk, dv, None, None
 
@@ -401,11 +401,11 @@ def create_dflash_mask(document_ids: torch.Tensor, total_seq_len: int,
     bounds = torch.empty(4, n_q, device=dev, dtype=torch.int32)
     scratch = torch.empty(total_seq_len, device=dev, dtype=torch.int32)
     causal_block = sliding_window is not None and not sliding_window_non_causal
-    _lib.call("spx_dflash_row_ranges", _lib.ptr(doc), _lib.kind_code(doc), total_seq_len,
-              _lib.ptr(anchors), _lib.kind_code(anchors), anchors.numel(), int(block_size),
+    _lib.call("spx_dflash_row_ranges", doc, _lib.kind_code(doc), total_seq_len,
+              anchors, _lib.kind_code(anchors), anchors.numel(), int(block_size),
               int(sliding_window) if sliding_window else 0, int(causal_block),
-              _lib.ptr(bounds[0]), _lib.ptr(bounds[1]), _lib.ptr(bounds[2]), _lib.ptr(bounds[3]),
-              _lib.ptr(scratch), _lib.stream_ptr(dev))
+              bounds[0], bounds[1], bounds[2], bounds[3],
+              scratch, _lib.stream_ptr(dev))
     return DFlashMask(bounds[0], bounds[1], bounds[2], bounds[3], total_seq_len, n_q)
 
 
@@ -426,12 +426,12 @@ class _DFlashAttention(torch.autograd.Function):
         dev = q.device
         out = torch.empty(1, nq, hq, d, device=dev, dtype=torch.bfloat16)
         lse = torch.empty(hq, nq, device=dev, dtype=torch.float32)
-        nbytes = int(_lib.load().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 0))
+        nbytes = int(_lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 0))
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_fwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(mask.ctx_lo), _lib.ptr(mask.ctx_hi),
-                  _lib.ptr(mask.blk_lo), _lib.ptr(mask.blk_hi), t, nq, hq, hkv, d, float(scaling),
-                  _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev))
+        _lib.call("spx_dflash_attn_fwd", q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), mask.ctx_lo, mask.ctx_hi,
+                  mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling),
+                  out, lse, ws, ws.numel(), _lib.stream_ptr(dev))
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.mask, ctx.scaling = mask, float(scaling)
         return out
@@ -446,13 +446,13 @@ class _DFlashAttention(torch.autograd.Function):
         dev = q.device
         dout = dout.to(torch.bfloat16).contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        nbytes = int(_lib.load().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 1))
+        nbytes = int(_lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 1))
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_bwd", _lib.ptr(q), q.stride(1), _lib.ptr(k), k.stride(1),
-                  _lib.ptr(v), v.stride(1), _lib.ptr(out), _lib.ptr(dout), _lib.ptr(lse),
-                  _lib.ptr(mask.ctx_lo), _lib.ptr(mask.ctx_hi), _lib.ptr(mask.blk_lo),
-                  _lib.ptr(mask.blk_hi), t, nq, hq, hkv, d, ctx.scaling, _lib.ptr(dq), dq.stride(1),
-                  _lib.ptr(dk), dk.stride(1), _lib.ptr(dv), dv.stride(1), _lib.ptr(ws), ws.numel(),
+        _lib.call("spx_dflash_attn_bwd", q, q.stride(1), k, k.stride(1),
+                  v, v.stride(1), out, dout, lse,
+                  mask.ctx_lo, mask.ctx_hi, mask.blk_lo,
+                  mask.blk_hi, t, nq, hq, hkv, d, ctx.scaling, dq, dq.stride(1),
+                  dk, dk.stride(1), dv, dv.stride(1), ws, ws.numel(),
                   _lib.stream_ptr(dev))
         return dq, dk, dv, None, None
 

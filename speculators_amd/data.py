@@ -28,6 +28,7 @@ Every layout also returns ``input_ids``, ``loss_mask``, ``position_ids`` and
 
 from __future__ import annotations
 
+import ctypes
 import json
 import os
 import queue
@@ -314,11 +315,12 @@ class BatchPacker:
                     slot.hs[at:at + keep].copy_(hs[:keep])
                     hs_seg.append((dst, dst, 0, n, -1))
             segments = ids_seg + hs_seg
+            table = (_lib.StageSegment * len(segments))(*segments)
             first = jobs[0][1] * row_bytes
             nbytes = (jobs[-1][1] + jobs[-1][2]) * row_bytes - first
             try:
-                _lib.call("spx_stage_upload", (_lib.StageSegment * len(segments))(*segments), len(segments),
-                          hs0 + first, _lib.ptr(slot.d_hs) + first, nbytes, self.copy_threads,
+                _lib.call("spx_stage_upload", ctypes.addressof(table), len(segments),
+                          hs0 + first, slot.d_hs.data_ptr() + first, nbytes, self.copy_threads,
                           self.stream.cuda_stream)
             except _lib.SpxError as exc:
                 raise OSError(str(exc)) if fds else exc
@@ -339,11 +341,11 @@ class BatchPacker:
             ints = torch.empty(3, 1, t, device=dev, dtype=torch.int64)
             ids, pos, doc = ints[0], ints[1], ints[2]
             mask = torch.empty(1, t, device=dev, dtype=self.mask_dtype)
-            _lib.call("spx_pack_batch", _lib.ptr(slot.d_hs), _lib.dtype_code(slot.d_hs), n,
-                      self.layers, h, _lib.ptr(slot.d_ids), _lib.ptr(slot.d_mask),
-                      slot.d_mask.element_size(), None, _lib.ptr(slot.d_plan[0]),
-                      _lib.ptr(slot.d_plan[1]), slot.n_docs, t, self.shift, _lib.ptr(aux),
-                      _lib.ptr(last), _lib.ptr(ids), _lib.ptr(mask), _lib.ptr(pos), _lib.ptr(doc),
+            _lib.call("spx_pack_batch", slot.d_hs, _lib.dtype_code(slot.d_hs), n,
+                      self.layers, h, slot.d_ids, slot.d_mask,
+                      slot.d_mask.element_size(), None, slot.d_plan[0],
+                      slot.d_plan[1], slot.n_docs, t, self.shift, aux,
+                      last, ids, mask, pos, doc,
                       self.stream.cuda_stream)
             slot.done.record(self.stream)
         slot.free.set()

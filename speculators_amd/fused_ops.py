@@ -29,8 +29,8 @@ class _RMSNorm(torch.autograd.Function):
         y = torch.empty(rows, h, device=x.device, dtype=torch.bfloat16)
         rstd = torch.empty(rows, device=x.device, dtype=torch.float32)
         w = weight.contiguous()
-        _lib.call("spx_rmsnorm_fwd", _lib.ptr(x2), x2.stride(0), _lib.ptr(w), _lib.ptr(y), h,
-                  _lib.ptr(rstd), rows, h, float(eps), _lib.stream_ptr(x.device))
+        _lib.call("spx_rmsnorm_fwd", x2, x2.stride(0), w, y, h,
+                  rstd, rows, h, float(eps), _lib.stream_ptr(x.device))
         ctx.save_for_backward(x2, w, rstd)
         ctx.shape = x.shape
         ctx.gain_grads = getattr(weight, "spx_gain_grads", None)
@@ -53,7 +53,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 def _dw_buffers(rows: int, h: int, device):
-    slots = int(_lib.load().spx_rmsnorm_bwd_slots(rows, h))
+    slots = int(_lib.native().spx_rmsnorm_bwd_slots(rows, h))
     return (torch.empty(slots * h, device=device, dtype=torch.float32),
             torch.empty(h, device=device, dtype=torch.bfloat16))
 
@@ -75,7 +75,7 @@ class GainGrads:
         task = torch._C._current_graph_task_id()
         if task != self.task:  # a pass that never reached the staging node leaves nothing behind
             self.scratch, self.marked, self.task = None, False, task
-        slots = int(_lib.load().spx_rmsnorm_bwd_slots(rows, h))
+        slots = int(_lib.native().spx_rmsnorm_bwd_slots(rows, h))
         if self.scratch is None:
             self.scratch = torch.empty(slots * h, device=device, dtype=torch.float32)
             self.slots, self.h = slots, h
@@ -90,7 +90,7 @@ class GainGrads:
         if self.marked:
             return None
         self.marked = True
-        return torch.zeros(1, device=device, dtype=torch.bfloat16).expand(self.h)
+        return _lib.zero(device, torch.bfloat16).expand(self.h)
 
     def finish(self):
         """The summed gradient (bf16 ``[H]``) of the uses recorded since the last call, or None."""
@@ -98,7 +98,7 @@ class GainGrads:
         if scratch is None:
             return None
         dw = torch.empty(self.h, device=scratch.device, dtype=torch.bfloat16)
-        _lib.call("spx_rmsnorm_dweight", _lib.ptr(scratch), self.slots, self.h, _lib.ptr(dw),
+        _lib.call("spx_rmsnorm_dweight", scratch, self.slots, self.h, dw,
                   _lib.stream_ptr(scratch.device))
         return dw
 
@@ -111,20 +111,20 @@ def _norm_backward(grads, need_dw, x, w, dy, dres, rstd, dx, rows, h):
     if need_dw and grads is not None:
         tgt = grads.target(rows, h, dev)
         if tgt is not None:
-            _lib.call("spx_rmsnorm_bwd_partial", _lib.ptr(x), x.stride(0), _lib.ptr(w), _lib.ptr(dy),
-                      dy.stride(0), _lib.ptr(dres), ld_dres, _lib.ptr(rstd), _lib.ptr(dx), h,
-                      _lib.ptr(tgt[0]), tgt[1], rows, h, st)
+            _lib.call("spx_rmsnorm_bwd_partial", x, x.stride(0), w, dy,
+                      dy.stride(0), dres, ld_dres, rstd, dx, h,
+                      tgt[0], tgt[1], rows, h, st)
             return grads.mark(dev)
     scratch = dw = None
     if need_dw:
         scratch, dw = _dw_buffers(rows, h, dev)
     if dres is not None:
-        _lib.call("spx_add_rmsnorm_bwd", _lib.ptr(x), x.stride(0), _lib.ptr(w), _lib.ptr(dy), dy.stride(0),
-                  _lib.ptr(dres), ld_dres, _lib.ptr(rstd), _lib.ptr(dx), h, _lib.ptr(dw), _lib.ptr(scratch),
+        _lib.call("spx_add_rmsnorm_bwd", x, x.stride(0), w, dy, dy.stride(0),
+                  dres, ld_dres, rstd, dx, h, dw, scratch,
                   rows, h, st)
     else:
-        _lib.call("spx_rmsnorm_bwd", _lib.ptr(x), x.stride(0), _lib.ptr(w), _lib.ptr(dy), dy.stride(0),
-                  _lib.ptr(rstd), _lib.ptr(dx), h, _lib.ptr(dw), _lib.ptr(scratch), rows, h, st)
+        _lib.call("spx_rmsnorm_bwd", x, x.stride(0), w, dy, dy.stride(0),
+                  rstd, dx, h, dw, scratch, rows, h, st)
     return dw
 
 
@@ -147,8 +147,8 @@ class _AddRMSNorm(torch.autograd.Function):
             torch.empty(rows, h, device=a.device, dtype=torch.bfloat16)
         rstd = torch.empty(rows, device=a.device, dtype=torch.float32)
         w = weight.contiguous()
-        _lib.call("spx_add_rmsnorm_fwd", _lib.ptr(a2), a2.stride(0), _lib.ptr(b2), b2.stride(0),
-                  _lib.ptr(s), h, _lib.ptr(w), _lib.ptr(y), h, _lib.ptr(rstd), rows, h, float(eps),
+        _lib.call("spx_add_rmsnorm_fwd", a2, a2.stride(0), b2, b2.stride(0),
+                  s, h, w, y, h, rstd, rows, h, float(eps),
                   _lib.stream_ptr(a.device))
         ctx.save_for_backward(s, w, rstd)
         ctx.shape = a.shape
@@ -216,10 +216,10 @@ class _PairNormCat(torch.autograd.Function):
         ctx.gain_grads = (getattr(wa, "spx_gain_grads", None), getattr(wb, "spx_gain_grads", None))
         wa, wb = wa.contiguous(), wb.contiguous()
         st = _lib.stream_ptr(a.device)
-        _lib.call("spx_rmsnorm_fwd", _lib.ptr(a2), a2.stride(0), _lib.ptr(wa), _lib.ptr(out), 2 * h,
-                  _lib.ptr(rstd[0]), rows, h, float(eps), st)
-        _lib.call("spx_rmsnorm_fwd", _lib.ptr(b2), b2.stride(0), _lib.ptr(wb), _lib.ptr(out[:, h:]), 2 * h,
-                  _lib.ptr(rstd[1]), rows, h, float(eps), st)
+        _lib.call("spx_rmsnorm_fwd", a2, a2.stride(0), wa, out, 2 * h,
+                  rstd[0], rows, h, float(eps), st)
+        _lib.call("spx_rmsnorm_fwd", b2, b2.stride(0), wb, out[:, h:], 2 * h,
+                  rstd[1], rows, h, float(eps), st)
         ctx.save_for_backward(a2, b2, wa, wb, rstd)
         ctx.shapes = (a.shape, b.shape)
         cat = out.view(*a.shape[:-1], 2 * h)
@@ -268,7 +268,7 @@ def rope_call(x_ptr, ld_x, x_head_stride, position_ids, inv_freq, out_ptr, ld_ou
     """One launch of the rotary relayout kernel; the rotated part of a head is what the frequency
     table covers (all of it, or its first ``2 * len(inv_freq)`` elements)."""
     rot = 2 * inv_freq.numel() if rotate else d
-    _lib.call("spx_rope_relayout_partial", x_ptr, ld_x, x_head_stride, _lib.ptr(position_ids), _lib.ptr(inv_freq),
+    _lib.call("spx_rope_relayout_partial", x_ptr, ld_x, x_head_stride, position_ids, inv_freq,
               out_ptr, ld_out, t, heads, d, rot, int(rotate), int(inverse), int(offset), float(table_scale),
               stream)
 
@@ -289,7 +289,7 @@ class _RopeRelayout(torch.autograd.Function):
             x2 = x2.contiguous()
         scale = table_scale_of(inv_freq)
         out = torch.empty(1, heads, t, d, device=x.device, dtype=torch.bfloat16)
-        rope_call(_lib.ptr(x2), x2.stride(0), d, position_ids, inv_freq, _lib.ptr(out), 0, t, heads, d, rotate,
+        rope_call(x2, x2.stride(0), d, position_ids, inv_freq, out, 0, t, heads, d, rotate,
                   0, offset, scale, _lib.stream_ptr(x.device))
         ctx.save_for_backward(position_ids, inv_freq)
         ctx.meta = (x.shape, heads, d, t, rotate, offset, scale)
@@ -301,7 +301,7 @@ class _RopeRelayout(torch.autograd.Function):
         shape, heads, d, t, rotate, offset, scale = ctx.meta
         dout = dout.to(torch.bfloat16).contiguous()
         dx = torch.empty(t, heads * d, device=dout.device, dtype=torch.bfloat16)
-        rope_call(_lib.ptr(dout), 0, d, position_ids, inv_freq, _lib.ptr(dx), heads * d, t, heads, d, rotate, 1,
+        rope_call(dout, 0, d, position_ids, inv_freq, dx, heads * d, t, heads, d, rotate, 1,
                   offset, scale, _lib.stream_ptr(dout.device))
         return dx.view(shape), None, None, None, None, None
 
@@ -349,8 +349,8 @@ class _SigmoidGate(torch.autograd.Function):
         if gate.stride(2) != 1:
             gate = gate.contiguous()
         y = torch.empty(t, heads * d, device=o.device, dtype=torch.bfloat16)
-        _lib.call("spx_sigmoid_gate_fwd", _lib.ptr(o2), o2.stride(0), _lib.ptr(gate), gate.stride(0),
-                  gate.stride(1), _lib.ptr(y), heads * d, t, heads, d, _lib.stream_ptr(o.device))
+        _lib.call("spx_sigmoid_gate_fwd", o2, o2.stride(0), gate, gate.stride(0),
+                  gate.stride(1), y, heads * d, t, heads, d, _lib.stream_ptr(o.device))
         ctx.save_for_backward(o2, gate)
         ctx.o_shape = o.shape
         return y.view(o.shape)
@@ -364,8 +364,8 @@ class _SigmoidGate(torch.autograd.Function):
             dy2 = dy2.contiguous()
         d_o = torch.empty(t, heads * d, device=dy.device, dtype=torch.bfloat16)
         dgate = torch.empty(t, heads, d, device=dy.device, dtype=torch.bfloat16)
-        _lib.call("spx_sigmoid_gate_bwd", _lib.ptr(o2), o2.stride(0), _lib.ptr(gate), gate.stride(0),
-                  gate.stride(1), _lib.ptr(dy2), dy2.stride(0), _lib.ptr(d_o), heads * d, _lib.ptr(dgate),
+        _lib.call("spx_sigmoid_gate_bwd", o2, o2.stride(0), gate, gate.stride(0),
+                  gate.stride(1), dy2, dy2.stride(0), d_o, heads * d, dgate,
                   heads * d, d, t, heads, d, _lib.stream_ptr(dy.device))
         return d_o.view(ctx.o_shape), dgate
 
@@ -537,7 +537,7 @@ class _SwiGLU(torch.autograd.Function):
         _need_bf16(gate, up)
         gate, up = gate.contiguous(), up.contiguous()
         out = torch.empty_like(gate)
-        _lib.call("spx_swiglu_fwd", _lib.ptr(gate), _lib.ptr(up), _lib.ptr(out), gate.numel(),
+        _lib.call("spx_swiglu_fwd", gate, up, out, gate.numel(),
                   _lib.stream_ptr(gate.device))
         ctx.save_for_backward(gate, up)
         return out
@@ -547,8 +547,8 @@ class _SwiGLU(torch.autograd.Function):
         gate, up = ctx.saved_tensors
         dout = dout.to(torch.bfloat16).contiguous()
         dg, du = torch.empty_like(gate), torch.empty_like(up)
-        _lib.call("spx_swiglu_bwd", _lib.ptr(gate), _lib.ptr(up), _lib.ptr(dout), _lib.ptr(dg),
-                  _lib.ptr(du), gate.numel(), _lib.stream_ptr(gate.device))
+        _lib.call("spx_swiglu_bwd", gate, up, dout, dg,
+                  du, gate.numel(), _lib.stream_ptr(gate.device))
         return dg, du
 
 

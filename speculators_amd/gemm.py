@@ -80,13 +80,13 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
         # (the kernel decides from the same numbers; here only whether the workspace is handed over)
         rem = (-(-m // 256) * -(-n // 256)) % _CUS
         if TAIL_PARTS > 1 and 0 < rem <= _CUS // 2 and k >= 64 * 16 * 2 and a.is_cuda:
-            nbytes = _lib.load().spx_gemm_tail_workspace_bytes()
+            nbytes = _lib.native().spx_gemm_tail_workspace_bytes()
             ws = _split_workspace(a.device, nbytes // 4)
-            _lib.call("spx_gemm_bf16_nt_tail", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
-                      _lib.ptr(out), out.stride(0), m, n, k, TAIL_PARTS, _lib.ptr(ws), nbytes, st)
+            _lib.call("spx_gemm_bf16_nt_tail", a, a.stride(0), b, b.stride(0),
+                      out, out.stride(0), m, n, k, TAIL_PARTS, ws, nbytes, st)
             return out
-        _lib.call("spx_gemm_bf16_nt", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
-                  _lib.ptr(out), out.stride(0), m, n, k, st)
+        _lib.call("spx_gemm_bf16_nt", a, a.stride(0), b, b.stride(0),
+                  out, out.stride(0), m, n, k, st)
     else:
         if m_live.dtype != torch.int32 or m_live.numel() != 1 or m_live.device != a.device:
             raise ValueError("m_live must be a one-element int32 tensor on the operands' device")
@@ -94,12 +94,12 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
         few_tiles = -(-m // 256) * -(-n // 256) <= 2 * 256
         if split and SPLIT_PARTS > 1 and few_tiles and n % 8 == 0 and out.stride(0) % 8 == 0 and k >= 64 * 16 * 2:
             ws = _split_workspace(a.device, SPLIT_PARTS * m * n)
-            _lib.call("spx_gemm_bf16_nt_rows_split", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
-                      _lib.ptr(out), out.stride(0), m, n, k, _lib.ptr(m_live), SPLIT_PARTS, _lib.ptr(ws),
+            _lib.call("spx_gemm_bf16_nt_rows_split", a, a.stride(0), b, b.stride(0),
+                      out, out.stride(0), m, n, k, m_live, SPLIT_PARTS, ws,
                       SPLIT_PARTS * m * n * 4, st)
         else:
-            _lib.call("spx_gemm_bf16_nt_rows", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
-                      _lib.ptr(out), out.stride(0), m, n, k, _lib.ptr(m_live), st)
+            _lib.call("spx_gemm_bf16_nt_rows", a, a.stride(0), b, b.stride(0),
+                      out, out.stride(0), m, n, k, m_live, st)
     return out
 
 
@@ -116,8 +116,8 @@ def _auto(form: int, a, b, out, m: int, n: int, k: int, ws_numel: int, m_live=No
     if out is None:
         out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
     ws = _split_workspace(a.device, ws_numel) if ws_numel else None
-    _lib.call("spx_gemm_bf16_auto", form, _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0), _lib.ptr(out),
-              out.stride(0), m, n, k, _lib.ptr(m_live), TAIL_PARTS, _lib.ptr(ws), ws_numel * 4,
+    _lib.call("spx_gemm_bf16_auto", form, a, a.stride(0), b, b.stride(0), out,
+              out.stride(0), m, n, k, m_live, TAIL_PARTS, ws, ws_numel * 4,
               _lib.stream_ptr(a.device))
     return out
 
@@ -192,10 +192,10 @@ def gemm_nt_stats(a: torch.Tensor, b: torch.Tensor, store: bool = True, want_arg
         raise ValueError("gemm_nt_stats: ask for the log-sum-exp, the arg-max or both")
     lse = torch.empty(m, device=dev, dtype=torch.float32) if want_lse else None
     am = torch.empty(m, device=dev, dtype=torch.int32) if want_argmax else None
-    nbytes = _lib.load().spx_gemm_stats_workspace_bytes(m, n)
+    nbytes = _lib.native().spx_gemm_stats_workspace_bytes(m, n)
     ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
-    _lib.call("spx_gemm_bf16_nt_stats", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0),
-              _lib.ptr(out), out.stride(0) if store else 0, m, n, k, _lib.ptr(lse), _lib.ptr(am), _lib.ptr(ws),
+    _lib.call("spx_gemm_bf16_nt_stats", a, a.stride(0), b, b.stride(0),
+              out, out.stride(0) if store else 0, m, n, k, lse, am, ws,
               nbytes, _lib.stream_ptr(dev))
     return out, lse, am
 
@@ -255,8 +255,8 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
         step = -(-t // bands)
         off = _band_offsets(t, step, bands, a.device)
         part = torch.empty(bands, m, n, device=a.device, dtype=torch.float32)
-        _lib.call("spx_gemm_bf16_tn_grouped", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0), _lib.ptr(part),
-                  n, m * n, m, n, t, _lib.ptr(off), bands, 1, 0, _lib.stream_ptr(a.device))
+        _lib.call("spx_gemm_bf16_tn_grouped", a, a.stride(0), b, b.stride(0), part,
+                  n, m * n, m, n, t, off, bands, 1, 0, _lib.stream_ptr(a.device))
         total = part.sum(0)
         if accumulate:
             total += out  # in fp32: what the result holds is added before the one rounding
@@ -269,8 +269,8 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
     st = _lib.stream_ptr(a.device)
     for t0 in range(0, t, rows):
         at, bt = a[t0:t0 + rows], b[t0:t0 + rows]
-        _lib.call(entry, _lib.ptr(at), at.stride(0), _lib.ptr(bt), bt.stride(0),
-                  _lib.ptr(out), out.stride(0), m, n, at.shape[0], int(accumulate or t0 > 0), st)
+        _lib.call(entry, at, at.stride(0), bt, bt.stride(0),
+                  out, out.stride(0), m, n, at.shape[0], int(accumulate or t0 > 0), st)
     return out
 
 
@@ -425,7 +425,7 @@ class _QKVRope(torch.autograd.Function):
                 out = torch.empty(1, heads, t, d, device=x.device, dtype=torch.bfloat16)
                 head_stride = 0
             part = qkv[:, col:]
-            FO.rope_call(_lib.ptr(part), n, d, position_ids, inv_freq, _lib.ptr(out), head_stride, t, heads, d,
+            FO.rope_call(part, n, d, position_ids, inv_freq, out, head_stride, t, heads, d,
                          rotate, 0, offset, scale, st)
             outs.append(out)
             col += heads * d
@@ -455,7 +455,7 @@ class _QKVRope(torch.autograd.Function):
                 if not (g.stride(3) == 1 and g.stride(2) == d and g.stride(1) % 8 == 0
                         and g.stride(1) >= t * d and g.data_ptr() % 16 == 0):
                     g = g.contiguous()
-                FO.rope_call(_lib.ptr(g), g.stride(1), d, position_ids, inv_freq, _lib.ptr(part), n, t, heads, d,
+                FO.rope_call(g, g.stride(1), d, position_ids, inv_freq, part, n, t, heads, d,
                              rotate, 1, offset, scale, st)
             col += heads * d
         dx = dw = None
@@ -493,7 +493,7 @@ class _GateUpSwiGLU(torch.autograd.Function):
         rows = x2.shape[0]
         if out is None or out.shape != (rows, f) or not out.is_contiguous():
             out = torch.empty(rows, f, device=x.device, dtype=torch.bfloat16)
-        _lib.call("spx_swiglu_rows_fwd", _lib.ptr(gu), 2 * f, _lib.ptr(gu[:, f:]), 2 * f, _lib.ptr(out), f,
+        _lib.call("spx_swiglu_rows_fwd", gu, 2 * f, gu[:, f:], 2 * f, out, f,
                   rows, f, _lib.stream_ptr(x.device))
         ctx.save_for_backward(x2, gu, wcat)
         ctx.meta = (x.shape, f, staged)
@@ -511,8 +511,8 @@ class _GateUpSwiGLU(torch.autograd.Function):
         dgu = staged.dy_slot(ctx.slot, rows) if ctx.needs_input_grad[1] else None
         if dgu is None:
             dgu = torch.empty(rows, 2 * f, device=x2.device, dtype=torch.bfloat16)
-        _lib.call("spx_swiglu_rows_bwd", _lib.ptr(gu), 2 * f, _lib.ptr(gu[:, f:]), 2 * f, _lib.ptr(d2),
-                  d2.stride(0), _lib.ptr(dgu), 2 * f, _lib.ptr(dgu[:, f:]), 2 * f, rows, f,
+        _lib.call("spx_swiglu_rows_bwd", gu, 2 * f, gu[:, f:], 2 * f, d2,
+                  d2.stride(0), dgu, 2 * f, dgu[:, f:], 2 * f, rows, f,
                   _lib.stream_ptr(x2.device))
         dx = dw = None
         if ctx.needs_input_grad[0]:

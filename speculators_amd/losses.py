@@ -100,13 +100,13 @@ def fused_loss_forward(op: int, logits: torch.Tensor, targets: torch.Tensor, tar
             lse_t, am_t = target_stats[0].reshape(-1), target_stats[1].reshape(-1)
         g = step.gathered
         _lib.call(
-            "spx_vocab_loss_step_fwd", op, _lib.ptr(x), x.stride(0), _lib.ptr(y), y.stride(0),
-            _lib.ptr(step.d2t), y.shape[1] if gather else 0, _lib.ptr(g) if gather else None,
-            g.stride(0) if gather else 0, rows, vocab, _lib.dtype_code(x), _lib.ptr(stats[0]),
-            _lib.ptr(stats[1]), _lib.ptr(lse_t), _lib.ptr(stats[3]), _lib.ptr(arg[0]), _lib.ptr(am_t),
-            int(reuse), _lib.ptr(step.mask), _lib.kind_code(step.mask) if step.mask is not None else 0,
-            _lib.ptr(step.prev), _lib.kind_code(step.prev) if step.prev is not None else 0,
-            _lib.ptr(step.counts), _lib.stream_ptr(dev),
+            "spx_vocab_loss_step_fwd", op, x, x.stride(0), y, y.stride(0),
+            step.d2t, y.shape[1] if gather else 0, g if gather else None,
+            g.stride(0) if gather else 0, rows, vocab, _lib.dtype_code(x), stats[0],
+            stats[1], lse_t, stats[3], arg[0], am_t,
+            int(reuse), step.mask, _lib.kind_code(step.mask) if step.mask is not None else 0,
+            step.prev, _lib.kind_code(step.prev) if step.prev is not None else 0,
+            step.counts, _lib.stream_ptr(dev),
         )
         return stats[0], stats[1], lse_t, stats[3], arg[0], am_t, x, (g if gather else y)
     reuse = target_stats is not None and op in (OP_KL, OP_CE)
@@ -119,9 +119,9 @@ def fused_loss_forward(op: int, logits: torch.Tensor, targets: torch.Tensor, tar
         if lse_t.numel() != rows or am_t.numel() != rows or lse_t.stride(0) != 1 or am_t.stride(0) != 1:
             raise ValueError("target_stats must be contiguous [rows] tensors")
     _lib.call(
-        "spx_fused_vocab_loss_fwd", op, _lib.ptr(x), x.stride(0), _lib.ptr(y), y.stride(0),
-        rows, vocab, _lib.dtype_code(x), _lib.ptr(stats[0]), _lib.ptr(stats[1]),
-        _lib.ptr(lse_t), _lib.ptr(stats[3]), _lib.ptr(arg[0]), _lib.ptr(am_t), int(reuse),
+        "spx_fused_vocab_loss_fwd", op, x, x.stride(0), y, y.stride(0),
+        rows, vocab, _lib.dtype_code(x), stats[0], stats[1],
+        lse_t, stats[3], arg[0], am_t, int(reuse),
         _lib.stream_ptr(dev),
     )
     return stats[0], stats[1], lse_t, stats[3], arg[0], am_t, x, y
@@ -138,17 +138,17 @@ def _ce_without_targets(logits, target_stats, step):
         raise ValueError("target_stats must be contiguous [rows] tensors")
     if step is not None:
         _lib.call(
-            "spx_vocab_loss_step_fwd", OP_CE, _lib.ptr(x), x.stride(0), None, 0, None, 0, None, 0, rows, vocab,
-            _lib.dtype_code(x), _lib.ptr(stats[0]), _lib.ptr(stats[1]), _lib.ptr(lse_t), _lib.ptr(stats[3]),
-            _lib.ptr(arg[0]), _lib.ptr(am_t), 1, _lib.ptr(step.mask),
-            _lib.kind_code(step.mask) if step.mask is not None else 0, _lib.ptr(step.prev),
-            _lib.kind_code(step.prev) if step.prev is not None else 0, _lib.ptr(step.counts),
+            "spx_vocab_loss_step_fwd", OP_CE, x, x.stride(0), None, 0, None, 0, None, 0, rows, vocab,
+            _lib.dtype_code(x), stats[0], stats[1], lse_t, stats[3],
+            arg[0], am_t, 1, step.mask,
+            _lib.kind_code(step.mask) if step.mask is not None else 0, step.prev,
+            _lib.kind_code(step.prev) if step.prev is not None else 0, step.counts,
             _lib.stream_ptr(dev))
     else:
         _lib.call(
-            "spx_fused_vocab_loss_fwd", OP_CE, _lib.ptr(x), x.stride(0), None, 0, rows, vocab,
-            _lib.dtype_code(x), _lib.ptr(stats[0]), _lib.ptr(stats[1]), _lib.ptr(lse_t), _lib.ptr(stats[3]),
-            _lib.ptr(arg[0]), _lib.ptr(am_t), 1, _lib.stream_ptr(dev))
+            "spx_fused_vocab_loss_fwd", OP_CE, x, x.stride(0), None, 0, rows, vocab,
+            _lib.dtype_code(x), stats[0], stats[1], lse_t, stats[3],
+            arg[0], am_t, 1, _lib.stream_ptr(dev))
     return stats[0], stats[1], lse_t, stats[3], arg[0], am_t, x, None
 
 
@@ -186,10 +186,10 @@ class _FusedLoss(torch.autograd.Function):
         g = grad_rows.reshape(-1).to(torch.float32).contiguous()
         grad = torch.empty(full_rows, vocab, device=x.device, dtype=x.dtype)
         _lib.call(
-            "spx_fused_vocab_loss_bwd", ctx.op, _lib.ptr(x), x.stride(0), _lib.ptr(y),
+            "spx_fused_vocab_loss_bwd", ctx.op, x, x.stride(0), y,
             y.stride(0) if y is not None else 0, rows, vocab, _lib.dtype_code(x),
-            _lib.ptr(lse_d), _lib.ptr(lse_t), _lib.ptr(extra), _lib.ptr(am_t), _lib.ptr(g), None,
-            _lib.ptr(grad), grad.stride(0), _lib.stream_ptr(x.device),
+            lse_d, lse_t, extra, am_t, g, None,
+            grad, grad.stride(0), _lib.stream_ptr(x.device),
         )
         if full_rows > rows:
             grad[rows:].zero_()
@@ -202,16 +202,16 @@ def _packed_row_map(row_grad: torch.Tensor, labels: torch.Tensor | None = None, 
     r``, the others to -1.  One small kernel; the count stays on the device."""
     rows = row_grad.numel()
     out = torch.empty(rows + 1, device=row_grad.device, dtype=torch.int32)
-    _lib.call("spx_pack_row_map", _lib.ptr(row_grad), _lib.ptr(labels), int(ignore_index), rows,
-              _lib.ptr(out), _lib.ptr(out[rows:]), _lib.stream_ptr(row_grad.device))
+    _lib.call("spx_pack_row_map", row_grad, labels, int(ignore_index), rows,
+              out, out[rows:], _lib.stream_ptr(row_grad.device))
     return out[:rows], out[rows:]
 
 
 def _unpack_rows_scaled(packed: torch.Tensor, row_map: torch.Tensor, row_scale: torch.Tensor, total_rows: int):
     """``_unpack_rows`` with live row r multiplied by ``row_scale[r]`` (fp32) on its way."""
     out = torch.empty(total_rows, packed.shape[1], device=packed.device, dtype=packed.dtype)
-    _lib.call("spx_unpack_rows_scaled", _lib.ptr(packed), packed.stride(0), _lib.ptr(row_map), _lib.ptr(row_scale),
-              row_map.numel(), total_rows, packed.shape[1], _lib.ptr(out), out.stride(0),
+    _lib.call("spx_unpack_rows_scaled", packed, packed.stride(0), row_map, row_scale,
+              row_map.numel(), total_rows, packed.shape[1], out, out.stride(0),
               _lib.stream_ptr(packed.device))
     return out
 
@@ -249,12 +249,12 @@ def _loss_forward_with_grad(op, x, y, known, step):
         if lse_t.numel() != rows or am_t.numel() != rows or lse_t.stride(0) != 1 or am_t.stride(0) != 1:
             raise ValueError("target_stats must be contiguous [rows] tensors")
     _lib.call(
-        "spx_vocab_loss_step_fwd_grad", op, _lib.ptr(x), x.stride(0), _lib.ptr(y),
-        y.stride(0) if y is not None else 0, rows, vocab, _lib.ptr(stats[0]), _lib.ptr(stats[1]),
-        _lib.ptr(lse_t), _lib.ptr(stats[3]), _lib.ptr(arg[0]), _lib.ptr(am_t), int(known is not None),
-        _lib.ptr(step.mask), _lib.kind_code(step.mask), _lib.ptr(step.prev),
-        _lib.kind_code(step.prev) if step.prev is not None else 0, _lib.ptr(step.counts),
-        _lib.ptr(row_map), _lib.ptr(packed), packed.stride(0), _lib.stream_ptr(dev))
+        "spx_vocab_loss_step_fwd_grad", op, x, x.stride(0), y,
+        y.stride(0) if y is not None else 0, rows, vocab, stats[0], stats[1],
+        lse_t, stats[3], arg[0], am_t, int(known is not None),
+        step.mask, _lib.kind_code(step.mask), step.prev,
+        _lib.kind_code(step.prev) if step.prev is not None else 0, step.counts,
+        row_map, packed, packed.stride(0), _lib.stream_ptr(dev))
     return stats[0], lse_t, arg[0], am_t, packed, row_map, count
 
 
@@ -262,8 +262,8 @@ def _unpack_rows(packed: torch.Tensor, row_map: torch.Tensor, total_rows: int):
     """One row per position again: live rows from their packed slot, the others (and the rows past
     the map, up to ``total_rows``) zero.  Slots past the count are never read."""
     out = torch.empty(total_rows, packed.shape[1], device=packed.device, dtype=packed.dtype)
-    _lib.call("spx_unpack_rows", _lib.ptr(packed), packed.stride(0), _lib.ptr(row_map), row_map.numel(),
-              total_rows, packed.shape[1], _lib.ptr(out), out.stride(0), _lib.stream_ptr(packed.device))
+    _lib.call("spx_unpack_rows", packed, packed.stride(0), row_map, row_map.numel(),
+              total_rows, packed.shape[1], out, out.stride(0), _lib.stream_ptr(packed.device))
     return out
 
 
@@ -319,10 +319,10 @@ class _HeadFusedLoss(torch.autograd.Function):
         row_map, count = _packed_row_map(g)
         packed = torch.empty(rows, vocab, device=x.device, dtype=x.dtype)
         _lib.call(
-            "spx_fused_vocab_loss_bwd_packed", ctx.op, _lib.ptr(x), x.stride(0), _lib.ptr(y),
+            "spx_fused_vocab_loss_bwd_packed", ctx.op, x, x.stride(0), y,
             y.stride(0) if y is not None else 0, rows, vocab, _lib.dtype_code(x),
-            _lib.ptr(lse_d), _lib.ptr(lse_t), _lib.ptr(extra), _lib.ptr(am_t), _lib.ptr(g), None,
-            _lib.ptr(row_map), _lib.ptr(packed), packed.stride(0), _lib.stream_ptr(x.device),
+            lse_d, lse_t, extra, am_t, g, None,
+            row_map, packed, packed.stride(0), _lib.stream_ptr(x.device),
         )
         dx_packed = matmul_nt(packed, weight_t, m_live=count)
         return (_unpack_rows(dx_packed, row_map, ctx.total_rows), None, None, None, None, None,
@@ -457,9 +457,9 @@ class _LabelCE(torch.autograd.Function):
         rows, vocab = logits2d.shape
         dev = logits2d.device
         out = torch.empty(2, rows, device=dev, dtype=torch.float32)
-        _lib.call("spx_label_ce_fwd", _lib.ptr(logits2d), logits2d.stride(0), _lib.ptr(labels), rows,
-                  vocab, _lib.dtype_code(logits2d), int(ignore_index), _lib.ptr(out[0]),
-                  _lib.ptr(out[1]), None, _lib.stream_ptr(dev))
+        _lib.call("spx_label_ce_fwd", logits2d, logits2d.stride(0), labels, rows,
+                  vocab, _lib.dtype_code(logits2d), int(ignore_index), out[0],
+                  out[1], None, _lib.stream_ptr(dev))
         ctx.save_for_backward(logits2d, labels, out[1])
         ctx.ignore_index = int(ignore_index)
         return out[0]
@@ -470,9 +470,9 @@ class _LabelCE(torch.autograd.Function):
         rows, vocab = logits2d.shape
         g = grad_rows.to(torch.float32).contiguous()
         dlogits = torch.empty(rows, vocab, device=logits2d.device, dtype=logits2d.dtype)
-        _lib.call("spx_label_ce_bwd", _lib.ptr(logits2d), logits2d.stride(0), _lib.ptr(labels),
-                  _lib.ptr(lse), _lib.ptr(g), rows, vocab, _lib.dtype_code(logits2d),
-                  ctx.ignore_index, _lib.ptr(dlogits), dlogits.stride(0),
+        _lib.call("spx_label_ce_bwd", logits2d, logits2d.stride(0), labels,
+                  lse, g, rows, vocab, _lib.dtype_code(logits2d),
+                  ctx.ignore_index, dlogits, dlogits.stride(0),
                   _lib.stream_ptr(logits2d.device))
         return dlogits, None, None
 
@@ -513,16 +513,16 @@ class _HeadLabelCE(torch.autograd.Function):
             rows, vocab = logits.shape
             out = torch.empty(2, rows, device=logits.device, dtype=torch.float32)
             out[1] = lse
-            _lib.call("spx_label_ce_from_lse", _lib.ptr(logits), logits.stride(0), _lib.ptr(labels), rows,
-                      vocab, _lib.dtype_code(logits), int(ignore_index), _lib.ptr(out[1]), _lib.ptr(out[0]),
+            _lib.call("spx_label_ce_from_lse", logits, logits.stride(0), labels, rows,
+                      vocab, _lib.dtype_code(logits), int(ignore_index), out[1], out[0],
                       _lib.stream_ptr(logits.device))
         else:
             logits = matmul_nt(x2, weight)
             rows, vocab = logits.shape
             out = torch.empty(2, rows, device=logits.device, dtype=torch.float32)
-            _lib.call("spx_label_ce_fwd", _lib.ptr(logits), logits.stride(0), _lib.ptr(labels), rows,
-                      vocab, _lib.dtype_code(logits), int(ignore_index), _lib.ptr(out[0]),
-                      _lib.ptr(out[1]), None, _lib.stream_ptr(logits.device))
+            _lib.call("spx_label_ce_fwd", logits, logits.stride(0), labels, rows,
+                      vocab, _lib.dtype_code(logits), int(ignore_index), out[0],
+                      out[1], None, _lib.stream_ptr(logits.device))
         ctx.save_for_backward(logits, labels, out[1], weight_t)
         ctx.ignore_index = int(ignore_index)
         ctx.mark_non_differentiable(logits)
@@ -541,9 +541,9 @@ class _HeadLabelCE(torch.autograd.Function):
         g = grad_rows.to(torch.float32).contiguous()
         row_map, count = _packed_row_map(g, labels, ctx.ignore_index)
         packed = torch.empty(rows, vocab, device=logits.device, dtype=logits.dtype)
-        _lib.call("spx_label_ce_bwd_packed", _lib.ptr(logits), logits.stride(0), _lib.ptr(labels),
-                  _lib.ptr(lse), _lib.ptr(g), rows, vocab, _lib.dtype_code(logits), ctx.ignore_index,
-                  _lib.ptr(row_map), _lib.ptr(packed), packed.stride(0),
+        _lib.call("spx_label_ce_bwd_packed", logits, logits.stride(0), labels,
+                  lse, g, rows, vocab, _lib.dtype_code(logits), ctx.ignore_index,
+                  row_map, packed, packed.stride(0),
                   _lib.stream_ptr(logits.device))
         dx_packed = matmul_nt(packed, weight_t, m_live=count)
         return _unpack_rows(dx_packed, row_map, rows), None, None, None, None, None
@@ -595,7 +595,7 @@ def vocab_gather(full_logits: torch.Tensor, d2t: torch.Tensor) -> torch.Tensor:
     while done < rows:  # the gather grid carries rows in its y dimension
         n = min(rows - done, 65535)
         xs, os_ = x[done:done + n], out[done:done + n]
-        _lib.call("spx_vocab_gather", _lib.ptr(xs), x.stride(0), _lib.ptr(d2t), _lib.ptr(os_),
+        _lib.call("spx_vocab_gather", xs, x.stride(0), d2t, os_,
                   out.stride(0), n, vd, vt, _lib.dtype_code(x), _lib.stream_ptr(x.device))
         done += n
     return out.view(*full_logits.shape[:-1], vd)

@@ -37,16 +37,16 @@ class _StepReduce(torch.autograd.Function):
         row_weight = torch.empty(n, device=row_loss.device, dtype=torch.float32)
         if counts is not None:
             _lib.call(
-                "spx_ttt_step_mean", _lib.ptr(row_loss), _lib.ptr(mask),
-                _lib.kind_code(mask) if mask is not None else 0, n, float(weight), _lib.ptr(counts),
-                _lib.ptr(out), _lib.ptr(row_weight), _lib.stream_ptr(row_loss.device),
+                "spx_ttt_step_mean", row_loss, mask,
+                _lib.kind_code(mask) if mask is not None else 0, n, float(weight), counts,
+                out, row_weight, _lib.stream_ptr(row_loss.device),
             )
         else:
             _lib.call(
-                "spx_ttt_step_reduce", _lib.ptr(row_loss), _lib.ptr(am_d), _lib.ptr(am_t),
-                _lib.ptr(mask), _lib.kind_code(mask) if mask is not None else 0,
-                _lib.ptr(prev), _lib.kind_code(prev) if prev is not None else 0,
-                n, float(weight), _lib.ptr(out), _lib.ptr(row_weight),
+                "spx_ttt_step_reduce", row_loss, am_d, am_t,
+                mask, _lib.kind_code(mask) if mask is not None else 0,
+                prev, _lib.kind_code(prev) if prev is not None else 0,
+                n, float(weight), out, row_weight,
                 _lib.stream_ptr(row_loss.device),
             )
         ctx.save_for_backward(row_weight)
@@ -280,9 +280,9 @@ def argmax_rows(logits: torch.Tensor) -> torch.Tensor:
     out = torch.empty(max(rows, 1), device=dev, dtype=torch.int32)
     if rows:
         _lib.call(
-            "spx_fused_vocab_loss_fwd", L.OP_CE, _lib.ptr(x), x.stride(0), _lib.ptr(x),
-            x.stride(0), rows, vocab, _lib.dtype_code(x), _lib.ptr(scratch[0]),
-            _lib.ptr(scratch[1]), _lib.ptr(scratch[2]), _lib.ptr(scratch[3]), _lib.ptr(out),
+            "spx_fused_vocab_loss_fwd", L.OP_CE, x, x.stride(0), x,
+            x.stride(0), rows, vocab, _lib.dtype_code(x), scratch[0],
+            scratch[1], scratch[2], scratch[3], out,
             None, 0, _lib.stream_ptr(dev),
         )
     return out[:rows].to(torch.int64).view(logits.shape[:-1])
@@ -295,9 +295,9 @@ class _BlockReduce(torch.autograd.Function):
         row_loss = row_loss.reshape(-1).contiguous()
         row_weight = torch.empty(n, device=row_loss.device, dtype=torch.float32)
         _lib.call(
-            "spx_block_reduce", _lib.ptr(row_loss), _lib.ptr(am_d), _lib.ptr(am_t), _lib.ptr(mask),
-            _lib.kind_code(mask), _lib.ptr(pos_weight), n, int(block_size), _lib.ptr(out),
-            _lib.ptr(correct), _lib.ptr(total), _lib.ptr(row_weight),
+            "spx_block_reduce", row_loss, am_d, am_t, mask,
+            _lib.kind_code(mask), pos_weight, n, int(block_size), out,
+            correct, total, row_weight,
             _lib.stream_ptr(row_loss.device),
         )
         ctx.save_for_backward(row_weight)

@@ -35,10 +35,10 @@ def gemm_nt_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor,
     rows = a.shape[0]
     if out is None:
         out = torch.empty(rows, n, device=a.device, dtype=torch.bfloat16)
-    nbytes = int(_lib.load().spx_gemm_grouped_workspace_bytes(rows, groups))
+    nbytes = int(_lib.native().spx_gemm_grouped_workspace_bytes(rows, groups))
     ws = torch.empty(nbytes // 4, device=a.device, dtype=torch.int32)
-    _lib.call("spx_gemm_bf16_nt_grouped", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(1), b.stride(0),
-              _lib.ptr(out), out.stride(0), rows, n, k, _lib.ptr(offsets), groups, _lib.ptr(ws), nbytes,
+    _lib.call("spx_gemm_bf16_nt_grouped", a, a.stride(0), b, b.stride(1), b.stride(0),
+              out, out.stride(0), rows, n, k, offsets, groups, ws, nbytes,
               _lib.stream_ptr(a.device))
     return out
 
@@ -60,10 +60,10 @@ def gemm_nn_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor,
     rows = a.shape[0]
     if out is None:
         out = torch.empty(rows, n, device=a.device, dtype=torch.bfloat16)
-    nbytes = int(_lib.load().spx_gemm_grouped_workspace_bytes(rows, groups))
+    nbytes = int(_lib.native().spx_gemm_grouped_workspace_bytes(rows, groups))
     ws = torch.empty(nbytes // 4, device=a.device, dtype=torch.int32)
-    _lib.call("spx_gemm_bf16_nn_grouped", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(1), b.stride(0),
-              _lib.ptr(out), out.stride(0), rows, n, k, _lib.ptr(offsets), groups, _lib.ptr(ws), nbytes,
+    _lib.call("spx_gemm_bf16_nn_grouped", a, a.stride(0), b, b.stride(1), b.stride(0),
+              out, out.stride(0), rows, n, k, offsets, groups, ws, nbytes,
               _lib.stream_ptr(a.device))
     return out
 
@@ -86,8 +86,8 @@ def gemm_tn_grouped(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor, out
         a = a.contiguous()
     if b.stride(1) != 1:
         b = b.contiguous()
-    _lib.call("spx_gemm_bf16_tn_grouped", _lib.ptr(a), a.stride(0), _lib.ptr(b), b.stride(0), _lib.ptr(out),
-              out.stride(1), out.stride(0), m, n, a.shape[0], _lib.ptr(offsets), groups,
+    _lib.call("spx_gemm_bf16_tn_grouped", a, a.stride(0), b, b.stride(0), out,
+              out.stride(1), out.stride(0), m, n, a.shape[0], offsets, groups,
               int(out.dtype == torch.float32), int(accumulate), _lib.stream_ptr(a.device))
     return out
 
@@ -108,8 +108,8 @@ def gemm_tn_grouped_multi(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tenso
         raise ValueError(f"out must be a contiguous bf16 or fp32 [{g1 - 1}, {m}, {n}] tensor")
     if offsets.dtype != torch.int32 or not offsets.is_contiguous() or offsets.device != a.device:
         raise ValueError("offsets must be a contiguous int32 tensor on the operands' device")
-    _lib.call("spx_gemm_bf16_tn_grouped_multi", _lib.ptr(a), m, _lib.ptr(b), n, _lib.ptr(out), n, m * n, m, n,
-              rows, segments, _lib.ptr(offsets), g1 - 1, int(out.dtype == torch.float32), int(accumulate),
+    _lib.call("spx_gemm_bf16_tn_grouped_multi", a, m, b, n, out, n, m * n, m, n,
+              rows, segments, offsets, g1 - 1, int(out.dtype == torch.float32), int(accumulate),
               _lib.stream_ptr(a.device))
     return out
 
@@ -176,8 +176,8 @@ def gather_rows(x2: torch.Tensor, src_row: torch.Tensor, scale: torch.Tensor | N
     rows, h = src_row.numel(), x2.shape[1]
     if out is None:
         out = torch.empty(rows, h, device=x2.device, dtype=torch.bfloat16)
-    _lib.call("spx_moe_gather_rows", _lib.ptr(x2), x2.stride(0), x2.shape[0], _lib.ptr(src_row),
-              _lib.ptr(scale), _lib.ptr(out), h, rows, h, _lib.stream_ptr(x2.device))
+    _lib.call("spx_moe_gather_rows", x2, x2.stride(0), x2.shape[0], src_row,
+              scale, out, h, rows, h, _lib.stream_ptr(x2.device))
     return out
 
 
@@ -186,8 +186,8 @@ def combine_rows(sorted_rows: torch.Tensor, pos: torch.Tensor, weight: torch.Ten
     tokens, k = pos.shape
     h = sorted_rows.shape[1]
     out = torch.empty(tokens, h, device=sorted_rows.device, dtype=torch.bfloat16)
-    _lib.call("spx_moe_combine_rows", _lib.ptr(sorted_rows), sorted_rows.stride(0), sorted_rows.shape[0],
-              _lib.ptr(pos), _lib.ptr(weight), _lib.ptr(out), h, tokens, k, h,
+    _lib.call("spx_moe_combine_rows", sorted_rows, sorted_rows.stride(0), sorted_rows.shape[0],
+              pos, weight, out, h, tokens, k, h,
               _lib.stream_ptr(sorted_rows.device))
     return out
 
@@ -196,8 +196,8 @@ def pair_dot(a: torch.Tensor, sorted_rows: torch.Tensor, pos: torch.Tensor) -> t
     """``out[t, j] = <a[t], sorted_rows[pos[t, j]]>`` in fp32."""
     tokens, k = pos.shape
     out = torch.empty(tokens, k, device=a.device, dtype=torch.float32)
-    _lib.call("spx_moe_pair_dot", _lib.ptr(a), a.stride(0), _lib.ptr(sorted_rows), sorted_rows.stride(0),
-              sorted_rows.shape[0], _lib.ptr(pos), _lib.ptr(out), tokens, k, a.shape[1],
+    _lib.call("spx_moe_pair_dot", a, a.stride(0), sorted_rows, sorted_rows.stride(0),
+              sorted_rows.shape[0], pos, out, tokens, k, a.shape[1],
               _lib.stream_ptr(a.device))
     return out
 
@@ -229,10 +229,10 @@ def sort_pairs(idx: torch.Tensor, num_experts: int):
     ints = torch.empty(2 * pairs + num_experts + 1, device=dev, dtype=torch.int32)
     src_row, pos, offsets = ints[:pairs], ints[pairs:2 * pairs], ints[2 * pairs:]
     if idx.is_cuda and num_experts <= SORT_MAX_EXPERTS and pairs:
-        nbytes = int(_lib.load().spx_moe_sort_workspace_bytes(pairs, num_experts))
+        nbytes = int(_lib.native().spx_moe_sort_workspace_bytes(pairs, num_experts))
         ws = torch.empty(nbytes // 4, device=dev, dtype=torch.int32)
-        _lib.call("spx_moe_sort_pairs", _lib.ptr(idx), t, k, num_experts, _lib.ptr(order), _lib.ptr(src_row),
-                  _lib.ptr(pos), _lib.ptr(offsets), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev))
+        _lib.call("spx_moe_sort_pairs", idx, t, k, num_experts, order, src_row,
+                  pos, offsets, ws, nbytes, _lib.stream_ptr(dev))
         return order, src_row, pos.view(t, k), offsets
     # host tensors, and more experts than the kernel's counters hold in LDS
     flat = idx.reshape(-1)
@@ -274,7 +274,7 @@ class _ExpertsMLP(torch.autograd.Function):
         act = (torch.empty(rows, inter, device=x2.device, dtype=torch.bfloat16) if stack_dn is None
                else stack_dn.x_slot(use_dn))
         up = hid[:, inter:]
-        _lib.call("spx_swiglu_rows_fwd", _lib.ptr(hid), i2, _lib.ptr(up), i2, _lib.ptr(act), inter, rows,
+        _lib.call("spx_swiglu_rows_fwd", hid, i2, up, i2, act, inter, rows,
                   inter, st)
         ys = gemm_nt_grouped(act, w_dn, off)
         wts = scores.float().contiguous()
@@ -303,8 +303,8 @@ class _ExpertsMLP(torch.autograd.Function):
         dact = gemm_nn_grouped(dys, st_dn.w, off)
         dh = (stack_gu.dy_slot(use_gu) if stack_gu is not None and want_gu
               else torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16))
-        _lib.call("spx_swiglu_rows_bwd", _lib.ptr(hid), i2, _lib.ptr(hid[:, inter:]), i2, _lib.ptr(dact), inter,
-                  _lib.ptr(dh), i2, _lib.ptr(dh[:, inter:]), i2, rows, inter, st)
+        _lib.call("spx_swiglu_rows_bwd", hid, i2, hid[:, inter:], i2, dact, inter,
+                  dh, i2, dh[:, inter:], i2, rows, inter, st)
         dx = None
         if ctx.needs_input_grad[0]:
             dx = combine_rows(gemm_nn_grouped(dh, st_gu.w, off), pos, None)

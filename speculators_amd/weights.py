@@ -86,7 +86,7 @@ def transposed_copy(w: torch.Tensor) -> torch.Tensor:
         r, c = w.shape[-2], w.shape[-1]
         batches = w.shape[0] if w.dim() == 3 else 1
         out = torch.empty(*w.shape[:-2], c, r, device=w.device, dtype=w.dtype)
-        _lib.call("spx_transpose_bf16", _lib.ptr(w), c, r * c, _lib.ptr(out), r, r * c, r, c, batches,
+        _lib.call("spx_transpose_bf16", w, c, r * c, out, r, r * c, r, c, batches,
                   _lib.stream_ptr(w.device))
         return out
     return w.transpose(-1, -2).contiguous()
@@ -221,7 +221,7 @@ class Staged:
         if self._marked:
             return None
         self._marked = True
-        return torch.zeros(1, device=self.w.device, dtype=torch.float32).expand(self.w.shape)
+        return _lib.zero(self.w.device).expand(self.w.shape)
 
     def grad_buffer(self):
         """``(buffer, holds)``: the buffer of ``w``'s shape that uses which compute their weight
@@ -257,6 +257,13 @@ class Staged:
 
                 self._dys, self._live, self._marked = None, [], False
                 return gemm_tn(dy, x, out_dtype=torch.bfloat16)
+        if bf16_ok and acc is None and not runs and len(self._extras) == 1 and not self._finishers:
+            dy, x = self._extras[0]
+            if _tn_ok(dy) and _tn_ok(x):
+                from .gemm import gemm_tn
+
+                self._extras, self._marked = [], False
+                return gemm_tn(dy, x, out_dtype=torch.bfloat16)
         for r0, n in runs:
             acc = wgrad_product(self._dys[r0:r0 + n], self._xs[r0:r0 + n], acc)
         for dy2, x2 in self._extras:
@@ -283,7 +290,7 @@ class _Stage(torch.autograd.Function):
             w = params[0].detach()
         else:
             w = _cat_bf16(params)
-        token = torch.zeros(1, device=w.device, dtype=torch.float32).expand(w.shape)
+        token = _lib.zero(w.device).expand(w.shape)
         ctx.mark_non_differentiable(w)
         ctx.set_materialize_grads(False)
         return w, token
@@ -319,7 +326,7 @@ class _StageGain(torch.autograd.Function):
         ctx.grads, ctx.dtype = grads, p.dtype
         if plus_one:
             return (1.0 + p.detach().float()).to(torch.bfloat16)
-        return p.detach().to(torch.bfloat16) if p.dtype != torch.bfloat16 else p.detach().clone()
+        return p.detach().to(torch.bfloat16)
 
     @staticmethod
     def backward(ctx, g):

@@ -33,6 +33,24 @@ def test_library_exports_every_declared_symbol():
     assert set(_lib.SIGNATURES) | {"spx_version", "spx_last_error"} == set(_declared_symbols())
 
 
+def test_binding_module_has_every_entry_point():
+    import torch
+
+    from speculators_amd import _lib
+
+    native = _lib.native()
+    for name in _declared_symbols():
+        assert hasattr(native, name), name
+    with pytest.raises(_lib.SpxError, match="unknown loss op"):
+        _lib.call("spx_fused_vocab_loss_fwd", 99, None, 0, None, 0, 1, 8, 0, None, None, None, None, None, None, 0,
+                  None)
+    with pytest.raises(_lib.SpxError, match="CPU tensor"):
+        native.spx_rmsnorm_dweight(torch.zeros(8), 1, None, 8, None)
+    with pytest.raises(TypeError):
+        native.spx_rmsnorm_bwd_slots(1)
+    assert native.spx_rmsnorm_bwd_slots(4096, 2048) == _lib.load().spx_rmsnorm_bwd_slots(4096, 2048)
+
+
 def test_argument_errors_do_not_need_a_gpu():
     from speculators_amd import _lib
 
