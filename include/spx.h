@@ -486,6 +486,28 @@ int spx_rmsnorm_bwd_partial(const void* x, int64_t ld_x, const void* weight, con
 int spx_rmsnorm_dweight(const float* dw_scratch, int64_t slots, int64_t H, void* dweight,
                         void* stream);
 
+/* Two RMSNorms of one row count in one launch, written into the halves of y [rows, 2H] (row stride ld_y):
+ * y[:, :H] = norm(a), y[:, H:] = norm(b); rstd [2, rows].  The backward of both (dy as y; dres_b, may be null,
+ * is added to b's input gradient; da / db may be null: only the gain's gradient is wanted then) leaves the
+ * partial sums of the gains' gradients in scratch_a / scratch_b as spx_rmsnorm_bwd_partial does. */
+int spx_rmsnorm_pair_fwd(const void* a, int64_t ld_a, const void* weight_a, const void* b, int64_t ld_b,
+                         const void* weight_b, void* y, int64_t ld_y, float* rstd, int64_t rows, int64_t H,
+                         float eps, void* stream);
+int spx_rmsnorm_pair_bwd_partial(const void* a, int64_t ld_a, const void* weight_a, const void* b, int64_t ld_b,
+                                 const void* weight_b, const void* dy, int64_t ld_dy, const void* dres_b,
+                                 int64_t ld_dres, const float* rstd, void* da, void* db, int64_t ld_dx,
+                                 float* scratch_a, int32_t accumulate_a, float* scratch_b, int32_t accumulate_b,
+                                 int64_t rows, int64_t H, void* stream);
+
+/* The relayout below for a merged q/k/v projection tok [T, (hq + 2 hkv) * D] (row stride ld_tok) in one launch:
+ * q [hq, T, D] and k [hkv, T, D] rotated, v [hkv, T, D] moved, each with its head stride (>= T * D; k and v may be
+ * windows of a cache).  inverse != 0: from q / k / v (the gradients; a null one stands for zeros) into tok with the
+ * transposed rotation. */
+int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_stride, void* k, int64_t k_head_stride,
+                 void* v, int64_t v_head_stride, const int64_t* position_ids, const float* inv_freq, int64_t T,
+                 int32_t hq, int32_t hkv, int32_t D, int32_t rotary_dim, int32_t inverse,
+                 int64_t position_offset, float table_scale, void* stream);
+
 /* Rotary embedding fused with the head-major relayout that precedes attention
  * (apply_rotary_pos_emb + the view/transpose of LlamaAttention.forward; for
  * DFlash models/dflash/model_definitions.py:29-45):

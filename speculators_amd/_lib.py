@@ -56,6 +56,11 @@ SIGNATURES["spx_dflash_attn_bwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _
                                      _I64, _I32, _I32, _I32, _F, _P, _I64, _P, _I64, _P, _I64, _P,
                                      _I64, _P]
 SIGNATURES["spx_rmsnorm_fwd"] = [_P, _I64, _P, _P, _I64, _P, _I64, _I64, _F, _P]
+SIGNATURES["spx_rmsnorm_pair_fwd"] = [_P, _I64, _P, _P, _I64, _P, _P, _I64, _P, _I64, _I64, _F, _P]
+SIGNATURES["spx_rmsnorm_pair_bwd_partial"] = [_P, _I64, _P, _P, _I64, _P, _P, _I64, _P, _I64, _P, _P, _P, _I64, _P,
+                                              _I32, _P, _I32, _I64, _I64, _P]
+SIGNATURES["spx_rope_qkv"] = [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32,
+                              _I64, _F, _P]
 SIGNATURES["spx_rmsnorm_bwd_slots"] = [_I64, _I64]
 SIGNATURES["spx_rmsnorm_bwd"] = [_P, _I64, _P, _P, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _P]
 SIGNATURES["spx_add_rmsnorm_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P, _I64, _I64, _F, _P]

@@ -25,12 +25,16 @@ __device__ __forceinline__ u32x4 pack8f(const float v[8]) {
   return r;
 }
 
-__device__ __forceinline__ float block_sum_256(float v, float* lds) {
+template <int WAVES>
+__device__ __forceinline__ float block_sum(float v, float* lds) {
   v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
   __syncthreads();
-  return lds[0] + lds[1] + lds[2] + lds[3];
+  float s = lds[0];
+#pragma unroll
+  for (int i = 1; i < WAVES; ++i) s += lds[i];
+  return s;
 }
 
 // ---------------------------------------------------------------- RMSNorm
@@ -38,14 +42,31 @@ __device__ __forceinline__ float block_sum_256(float v, float* lds) {
 // wave per row (small H, e.g. per-head q/k norm).  MAXC = 16-byte chunks a lane keeps.
 // RES: x is the sum of two tensors, x = bf16(x + res) (one rounding, as a bf16 tensor add),
 // which is also written to `sum` for the residual stream.
-template <int MAXC, bool WAVE_ROWS, bool RES = false>
-__global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
-    const uint16_t* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
-    uint16_t* __restrict__ y, int64_t ld_y, float* __restrict__ rstd, int64_t rows, int H,
+// The kernel is bound by HBM where the rows fill the chip and by the launch below that: the two norms
+// of the first layer (PAIR) are one launch of twice the workgroups, the upper half of the grid's y
+// working on the second norm (T = 512, H = 2048: 3.7 us for the pair, 4.1 us for each one alone).
+struct NormFwdSet {
+  const uint16_t* x;
+  int64_t ld_x;
+  const uint16_t* w;
+  uint16_t* y;
+  int64_t ld_y;
+  float* rstd;
+};
+
+template <int MAXC, bool WAVE_ROWS, bool RES = false, bool PAIR = false, int NT = 256>
+__global__ __launch_bounds__(NT) void rmsnorm_fwd_kernel(
+    NormFwdSet one, NormFwdSet two, int64_t rows, int H,
     float eps, const uint16_t* __restrict__ res = nullptr, int64_t ld_res = 0,
     uint16_t* __restrict__ sum = nullptr, int64_t ld_sum = 0) {
-  __shared__ float red[4];
-  const int nthr = WAVE_ROWS ? 64 : 256;
+  __shared__ float red[NT / 64];
+  const bool second = PAIR && blockIdx.y;
+  const uint16_t* __restrict__ x = second ? two.x : one.x;
+  const uint16_t* __restrict__ w = second ? two.w : one.w;
+  uint16_t* __restrict__ y = second ? two.y : one.y;
+  float* __restrict__ rstd = second ? two.rstd : one.rstd;
+  const int64_t ld_x = second ? two.ld_x : one.ld_x, ld_y = second ? two.ld_y : one.ld_y;
+  const int nthr = WAVE_ROWS ? 64 : NT;
   const int t = WAVE_ROWS ? (threadIdx.x & 63) : threadIdx.x;
   const int64_t row = WAVE_ROWS ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   if (WAVE_ROWS && row >= rows) return;
@@ -70,7 +91,7 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
       for (int e = 0; e < 8; ++e) ss = fmaf(v[c][e], v[c][e], ss);
     }
   }
-  ss = WAVE_ROWS ? wave_sum(ss) : block_sum_256(ss, red);
+  ss = WAVE_ROWS ? wave_sum(ss) : block_sum<NT / 64>(ss, red);
   const float r = rsqrtf(ss / (float)H + eps);
   if (t == 0 && rstd) rstd[row] = r;
 #pragma unroll
@@ -91,14 +112,43 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
 // dres (may be null): gradient that reaches x along the residual stream, added before the
 // one rounding of dx.  dx may be null (only dw wanted).  accumulate: the partial sums start from
 // what dw_part holds (a gain that is applied several times per forward: one buffer, one final sum).
-template <int MAXC, bool WAVE_ROWS>
-__global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
-    const uint16_t* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
-    const uint16_t* __restrict__ dy, int64_t ld_dy, const float* __restrict__ rstd,
-    uint16_t* __restrict__ dx, int64_t ld_dx, float* __restrict__ dw_part, int64_t rows, int H,
-    const uint16_t* __restrict__ dres = nullptr, int64_t ld_dres = 0, int accumulate = 0) {
-  __shared__ float red[4];
-  const int nthr = WAVE_ROWS ? 64 : 256;
+// Bound by HBM (x, dy, dres in, dx out; the partial sums are 1024 rows of fp32, read and written).  A
+// lane keeps at most two 16-byte chunks of a row: with eight (wide rows on 256 threads) the four
+// arrays took 256 registers and 8192 x 8192 took 233 us (2.3 TB/s); 512 or 1024 threads share such a row
+// now: 106 us.
+// The narrow form (one wave per row) adds its four waves' sums through LDS: the final sum over the
+// slots has a quarter of the rows to read (a q / k norm of 128: 8192 slots before).
+// PAIR as in the forward: the upper half of the grid's y is the second norm.
+struct NormBwdSet {
+  const uint16_t* x;
+  int64_t ld_x;
+  const uint16_t* w;
+  const uint16_t* dy;
+  int64_t ld_dy;
+  const float* rstd;
+  uint16_t* dx;
+  int64_t ld_dx;
+  float* dw_part;
+  const uint16_t* dres;
+  int64_t ld_dres;
+  int accumulate;
+};
+
+template <int MAXC, bool WAVE_ROWS, bool PAIR = false, int NT = 256>
+__global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(NormBwdSet one, NormBwdSet two, int64_t rows, int H) {
+  __shared__ float red[WAVE_ROWS ? 4 * 512 : NT / 64];
+  const bool second = PAIR && blockIdx.y;
+  const uint16_t* __restrict__ x = second ? two.x : one.x;
+  const uint16_t* __restrict__ w = second ? two.w : one.w;
+  const uint16_t* __restrict__ dy = second ? two.dy : one.dy;
+  const float* __restrict__ rstd = second ? two.rstd : one.rstd;
+  uint16_t* __restrict__ dx = second ? two.dx : one.dx;
+  float* __restrict__ dw_part = second ? two.dw_part : one.dw_part;
+  const uint16_t* __restrict__ dres = second ? two.dres : one.dres;
+  const int64_t ld_x = second ? two.ld_x : one.ld_x, ld_dy = second ? two.ld_dy : one.ld_dy;
+  const int64_t ld_dx = second ? two.ld_dx : one.ld_dx, ld_dres = second ? two.ld_dres : one.ld_dres;
+  const int accumulate = second ? two.accumulate : one.accumulate;
+  const int nthr = WAVE_ROWS ? 64 : NT;
   const int t = WAVE_ROWS ? (threadIdx.x & 63) : threadIdx.x;
   const int wave = threadIdx.x >> 6;
   const int nch = H / 8;
@@ -109,9 +159,8 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
     if (ch < nch) unpack8f(*reinterpret_cast<const u32x4*>(w + ch * 8), wv[c]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) dwacc[c][e] = 0.f;
-    if (accumulate && dw_part && ch < nch) {
-      const int64_t slot0 = WAVE_ROWS ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
-      const float* o = dw_part + slot0 * H + ch * 8;
+    if (accumulate && dw_part && ch < nch && !(WAVE_ROWS && wave)) {
+      const float* o = dw_part + (int64_t)blockIdx.x * H + ch * 8;
       const f32x4 a = *reinterpret_cast<const f32x4*>(o), b = *reinterpret_cast<const f32x4*>(o + 4);
       dwacc[c][0] = a.x; dwacc[c][1] = a.y; dwacc[c][2] = a.z; dwacc[c][3] = a.w;
       dwacc[c][4] = b.x; dwacc[c][5] = b.y; dwacc[c][6] = b.z; dwacc[c][7] = b.w;
@@ -140,7 +189,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
       }
     }
     if (dx == nullptr) continue;  // uniform: only the weight gradient is wanted
-    dot = WAVE_ROWS ? wave_sum(dot) : block_sum_256(dot, red);
+    dot = WAVE_ROWS ? wave_sum(dot) : block_sum<NT / 64>(dot, red);
     const float mean = dot / (float)H;
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
@@ -160,12 +209,25 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
     }
   }
   if (dw_part) {
-    const int64_t slot = WAVE_ROWS ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
+    if (WAVE_ROWS) {
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c) {
+        const int ch = t + c * nthr;
+        if (ch < nch) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) red[wave * H + ch * 8 + e] = dwacc[c][e];
+        }
+      }
+      __syncthreads();
+      for (int c = threadIdx.x; c < H; c += NT)
+        dw_part[(int64_t)blockIdx.x * H + c] = (red[c] + red[H + c]) + (red[2 * H + c] + red[3 * H + c]);
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
       const int ch = t + c * nthr;
       if (ch < nch) {
-        float* o = dw_part + slot * H + ch * 8;
+        float* o = dw_part + (int64_t)blockIdx.x * H + ch * 8;
         f32x4 a = {dwacc[c][0], dwacc[c][1], dwacc[c][2], dwacc[c][3]};
         f32x4 b = {dwacc[c][4], dwacc[c][5], dwacc[c][6], dwacc[c][7]};
         *reinterpret_cast<f32x4*>(o) = a;
@@ -176,26 +238,38 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
 }
 
 // dw[c] = sum_s dw_part[s, c]  (fixed order: deterministic), bf16 out.  One workgroup
-// sums 32 columns (one 128-byte line per slot row): lane = (slot row j of 32, 4 columns),
-// thread j adds the slots j, j + 32, ..., then the 32 partial sums are combined through LDS
-// in a fixed order.
-__global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ part, int64_t slots,
-                                                     int H, uint16_t* __restrict__ out) {
-  __shared__ float red[32][33];
+// sums 32 columns (one 128-byte line per slot row): lane = (slot row j of 128, 4 columns),
+// thread j adds the slots j, j + 128, ..., then the 128 partial sums are combined through LDS
+// in a fixed order.  A latency-bound read of few megabytes by few workgroups: 1024 threads have
+// eight loads each to wait for at 1024 slots (256 threads had 32: 11.6 us at H = 4096, 3.5 us now).
+__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ part, int64_t slots,
+                                                      int H, uint16_t* __restrict__ out) {
+  __shared__ float red[128][33];
+  __shared__ float sub[8][33];
   const int q = threadIdx.x & 7, j = threadIdx.x >> 3;
   const int c = blockIdx.x * 32 + q * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  if (c < H)
-    for (int64_t i = j; i < slots; i += 32) {
+  if (c < H) {
+#pragma unroll 8
+    for (int64_t i = j; i < slots; i += 128) {
       const f32x4 v = *reinterpret_cast<const f32x4*>(part + i * H + c);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
+  }
   red[j][q * 4 + 0] = s.x; red[j][q * 4 + 1] = s.y; red[j][q * 4 + 2] = s.z; red[j][q * 4 + 3] = s.w;
+  __syncthreads();
+  const int col = threadIdx.x & 31, g = threadIdx.x >> 5;
+  if (g < 8) {
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t += red[g * 16 + k][col];
+    sub[g][col] = t;
+  }
   __syncthreads();
   if (threadIdx.x < 32 && blockIdx.x * 32 + threadIdx.x < H) {
     float t = 0.f;
 #pragma unroll
-    for (int k = 0; k < 32; ++k) t += red[k][threadIdx.x];
+    for (int k = 0; k < 8; ++k) t += sub[k][threadIdx.x];
     out[blockIdx.x * 32 + threadIdx.x] = (uint16_t)f32_to_bf16_bits(t);
   }
 }
@@ -238,8 +312,10 @@ __global__ __launch_bounds__(256) void rope_kernel(const uint16_t* __restrict__ 
     for (int e = 0; e < 8; ++e) {
       const float ang = p * inv_freq[d0 + e];
       // (table_scale: the attention factor some frequency scalings put on both tables, 1 otherwise)
-      const float c = round_bf16(cosf(ang) * table_scale);
-      float s = round_bf16(sinf(ang) * table_scale);
+      float sn, cs;
+      sincosf(ang, &sn, &cs);
+      const float c = round_bf16(cs * table_scale);
+      float s = round_bf16(sn * table_scale);
       if (INVERSE) s = -s;
       // x*cos + rotate_half(x)*sin with each bf16 op rounded
       oa[e] = round_bf16(a[e] * c) + round_bf16(-b[e] * s);
@@ -251,6 +327,98 @@ __global__ __launch_bounds__(256) void rope_kernel(const uint16_t* __restrict__ 
   }
   *reinterpret_cast<u32x4*>(dst + dA) = pack8f(oa);
   *reinterpret_cast<u32x4*>(dst + half + dA) = pack8f(ob);
+}
+
+// The relayout of a merged q/k/v projection [T, (hq + 2 hkv) * D] (row stride ld) in one launch: q and k
+// rotated, v moved.  Head-major sides [heads][T][D] with a head stride each (k and v may be windows of a
+// cache).  INVERSE: the other way with the transposed rotation; a null source is a gradient of zeros.
+// Bound by HBM, and by the evaluation of cos / sin where every head does its own: a thread works on the
+// same 16 elements of HEADS heads of one token (head i * groups + hg: neighbouring lanes stay on
+// neighbouring heads of the token-major row) and evaluates the angles once.  4096 tokens of 48 heads of
+// 128: 32 us, three launches of the kernel above 47 us; 512 tokens of 48 x 64: 6.0 us for 20.
+template <bool INVERSE, int HEADS>
+__global__ __launch_bounds__(256) void rope_qkv_kernel(uint16_t* __restrict__ tok, int64_t ld,
+                                                       uint16_t* __restrict__ q, int64_t hs_q,
+                                                       uint16_t* __restrict__ k, int64_t hs_k,
+                                                       uint16_t* __restrict__ v, int64_t hs_v,
+                                                       const int64_t* __restrict__ pos,
+                                                       const float* __restrict__ inv_freq, int T, int hq, int hkv,
+                                                       int D, int rot, int64_t pos_offset, float table_scale) {
+  const unsigned per_row = (unsigned)D / 16;
+  const int heads = hq + 2 * hkv;
+  const unsigned groups = (unsigned)(heads + HEADS - 1) / HEADS;
+  const unsigned item = blockIdx.x * 256u + threadIdx.x;
+  if (item >= (unsigned)T * groups * per_row) return;
+  const int d0 = (int)(item % per_row) * 8;
+  const unsigned rest = item / per_row;
+  const int hg = (int)(rest % groups);
+  const int t = (int)(rest / groups);
+  const bool pass = d0 * 2 >= rot;
+  const int half = pass ? 8 : rot / 2;
+  const int dA = pass ? d0 * 2 : d0;
+  u32x4 ra[HEADS], rb[HEADS];
+#pragma unroll
+  for (int i = 0; i < HEADS; ++i) {
+    const int h = i * (int)groups + hg;
+    ra[i] = u32x4{0, 0, 0, 0};
+    rb[i] = u32x4{0, 0, 0, 0};
+    if (h < heads) {
+      const uint16_t* src;
+      if (INVERSE) {
+        src = h < hq ? q : (h < hq + hkv ? k : v);
+        const int64_t hs = h < hq ? hs_q : (h < hq + hkv ? hs_k : hs_v);
+        const int hh = h < hq ? h : (h < hq + hkv ? h - hq : h - hq - hkv);
+        if (src) src += (int64_t)hh * hs + (int64_t)t * D;
+      } else {
+        src = tok + (int64_t)t * ld + h * D;
+      }
+      if (!INVERSE || src) {
+        ra[i] = *reinterpret_cast<const u32x4*>(src + dA);
+        rb[i] = *reinterpret_cast<const u32x4*>(src + half + dA);
+      }
+    }
+  }
+  float c[8], s[8];
+  if (!pass && hg < hq + hkv) {
+    const float p = (float)(pos[t] + pos_offset);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float ang = p * inv_freq[d0 + e];
+      float sn, cs;
+      sincosf(ang, &sn, &cs);  // one argument reduction for both
+      c[e] = round_bf16(cs * table_scale);
+      s[e] = round_bf16(sn * table_scale);
+      if (INVERSE) s[e] = -s[e];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < HEADS; ++i) {
+    const int h = i * (int)groups + hg;
+    if (h < heads) {
+      uint16_t* dst;
+      if (INVERSE) {
+        dst = tok + (int64_t)t * ld + h * D;
+      } else {
+        const int64_t hs = h < hq ? hs_q : (h < hq + hkv ? hs_k : hs_v);
+        const int hh = h < hq ? h : (h < hq + hkv ? h - hq : h - hq - hkv);
+        dst = (h < hq ? q : (h < hq + hkv ? k : v)) + (int64_t)hh * hs + (int64_t)t * D;
+      }
+      if (!pass && h < hq + hkv) {
+        float a[8], b[8], oa[8], ob[8];
+        unpack8f(ra[i], a);
+        unpack8f(rb[i], b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          oa[e] = round_bf16(a[e] * c[e]) + round_bf16(-b[e] * s[e]);
+          ob[e] = round_bf16(b[e] * c[e]) + round_bf16(a[e] * s[e]);
+        }
+        ra[i] = pack8f(oa);
+        rb[i] = pack8f(ob);
+      }
+      *reinterpret_cast<u32x4*>(dst + dA) = ra[i];
+      *reinterpret_cast<u32x4*>(dst + half + dA) = rb[i];
+    }
+  }
 }
 
 // out[b][c][r] = in[b][r][c] for a stack of bf16 matrices (the per-expert transposes the input
@@ -488,10 +656,21 @@ extern "C" int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, con
   return check_launch(__func__);
 }
 
+// one slot per workgroup, four workgroups per compute unit (narrow rows: one row per wave, eight)
 extern "C" int64_t spx_rmsnorm_bwd_slots(int64_t rows, int64_t H) {
-  if (H <= 512) return 4 * (rows < 8192 ? (rows + 3) / 4 : 2048);  // one wave per slot, 8 workgroups per CU
-  return rows < 1024 ? rows : 1024;  // four workgroups per compute unit
+  if (H <= 512) return rows < 8192 ? (rows + 3) / 4 : 2048;
+  return rows < 1024 ? rows : 1024;
 }
+
+// Threads per row: a lane keeps at most two chunks of 8 elements (see rmsnorm_bwd_kernel)
+#define SPX_NORM_FORMS(LAUNCH)                      \
+  do {                                              \
+    if (H <= 512) LAUNCH(1, true, 256);             \
+    else if (H <= 2048) LAUNCH(1, false, 256);      \
+    else if (H <= 4096) LAUNCH(2, false, 256);      \
+    else if (H <= 8192) LAUNCH(2, false, 512);      \
+    else LAUNCH(2, false, 1024);                    \
+  } while (0)
 
 static int rmsnorm_fwd_launch(const char* fn, const void* x, int64_t ld_x, const void* res, int64_t ld_res,
                               void* sum, int64_t ld_sum, const void* weight, void* y, int64_t ld_y,
@@ -506,23 +685,21 @@ static int rmsnorm_fwd_launch(const char* fn, const void* x, int64_t ld_x, const
   if (!(al16(x) && al16(weight) && al16(y) && al16(res) && al16(sum)))
     return fail_arg(fn, "buffers must be 16-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  auto xp = reinterpret_cast<const uint16_t*>(x);
   auto rp = reinterpret_cast<const uint16_t*>(res);
   auto sp = reinterpret_cast<uint16_t*>(sum);
-  auto wp = reinterpret_cast<const uint16_t*>(weight);
-  auto yp = reinterpret_cast<uint16_t*>(y);
-#define SPX_LAUNCH(MAXC, WR, GRID)                                                                  \
-  do {                                                                                              \
-    if (res)                                                                                        \
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, true>), dim3((unsigned)(GRID)), dim3(256), 0, st, \
-                         xp, ld_x, wp, yp, ld_y, rstd, rows, (int)H, eps, rp, ld_res, sp, ld_sum);  \
-    else                                                                                            \
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, false>), dim3((unsigned)(GRID)), dim3(256), 0, st, \
-                         xp, ld_x, wp, yp, ld_y, rstd, rows, (int)H, eps, nullptr, 0, nullptr, 0);  \
+  const NormFwdSet set = {reinterpret_cast<const uint16_t*>(x), ld_x, reinterpret_cast<const uint16_t*>(weight),
+                          reinterpret_cast<uint16_t*>(y), ld_y, rstd};
+#define SPX_LAUNCH(MAXC, WR, NT)                                                                             \
+  do {                                                                                                       \
+    const unsigned grid = (unsigned)(WR ? (rows + 3) / 4 : rows);                                            \
+    if (res)                                                                                                 \
+      hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, true, false, NT>), dim3(grid), dim3(NT), 0, st, set,  \
+                         set, rows, (int)H, eps, rp, ld_res, sp, ld_sum);                                    \
+    else                                                                                                     \
+      hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, false, false, NT>), dim3(grid), dim3(NT), 0, st, set, \
+                         set, rows, (int)H, eps, nullptr, 0, nullptr, 0);                                    \
   } while (0)
-  if (H <= 512) SPX_LAUNCH(1, true, (rows + 3) / 4);
-  else if (H <= 4096) SPX_LAUNCH(2, false, rows);
-  else SPX_LAUNCH(8, false, rows);
+  SPX_NORM_FORMS(SPX_LAUNCH);
 #undef SPX_LAUNCH
   return check_launch(fn);
 }
@@ -539,6 +716,29 @@ extern "C" int spx_add_rmsnorm_fwd(const void* a, int64_t ld_a, const void* b, i
   SPX_REQUIRE(rows == 0 || (b && sum), "null buffer");
   return rmsnorm_fwd_launch(__func__, a, ld_a, b, ld_b, sum, ld_sum, weight, y, ld_y, rstd, rows, H, eps,
                             stream);
+}
+
+extern "C" int spx_rmsnorm_pair_fwd(const void* a, int64_t ld_a, const void* weight_a, const void* b, int64_t ld_b,
+                                    const void* weight_b, void* y, int64_t ld_y, float* rstd, int64_t rows,
+                                    int64_t H, float eps, void* stream) {
+  SPX_REQUIRE(rows > 0 && rows < (1ll << 31) && H > 0 && H % 8 == 0 && H <= 16384,
+              "rows > 0 and H a multiple of 8, at most 16384");
+  SPX_REQUIRE(ld_a % 8 == 0 && ld_b % 8 == 0 && ld_y % 8 == 0 && ld_y >= 2 * H,
+              "the row strides must be multiples of 8, that of y at least 2 H");
+  SPX_REQUIRE(a && weight_a && b && weight_b && y && rstd, "null buffer");
+  SPX_REQUIRE(al16(a) && al16(weight_a) && al16(b) && al16(weight_b) && al16(y), "buffers must be 16-byte aligned");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  uint16_t* yp = reinterpret_cast<uint16_t*>(y);
+  const NormFwdSet one = {reinterpret_cast<const uint16_t*>(a), ld_a, reinterpret_cast<const uint16_t*>(weight_a),
+                          yp, ld_y, rstd};
+  const NormFwdSet two = {reinterpret_cast<const uint16_t*>(b), ld_b, reinterpret_cast<const uint16_t*>(weight_b),
+                          yp + H, ld_y, rstd + rows};
+#define SPX_LAUNCH(MAXC, WR, NT)                                                                                 \
+  hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, false, true, NT>), dim3((unsigned)(WR ? (rows + 3) / 4 : rows), 2), \
+                     dim3(NT), 0, st, one, two, rows, (int)H, eps, nullptr, 0, nullptr, 0)
+  SPX_NORM_FORMS(SPX_LAUNCH);
+#undef SPX_LAUNCH
+  return check_launch(__func__);
 }
 
 static int rmsnorm_bwd_launch(const char* fn, const void* x, int64_t ld_x, const void* weight, const void* dy,
@@ -558,26 +758,50 @@ static int rmsnorm_bwd_launch(const char* fn, const void* x, int64_t ld_x, const
   if (!(al16(x) && al16(weight) && al16(dy) && al16(dx) && al16(dw_scratch) && al16(dres)))
     return fail_arg(fn, "buffers must be 16-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  auto xp = reinterpret_cast<const uint16_t*>(x);
-  auto wp = reinterpret_cast<const uint16_t*>(weight);
-  auto dyp = reinterpret_cast<const uint16_t*>(dy);
-  auto drp = reinterpret_cast<const uint16_t*>(dres);
-  auto dxp = reinterpret_cast<uint16_t*>(dx);
   float* part = (dweight || partial_only) ? dw_scratch : nullptr;
+  const NormBwdSet set = {reinterpret_cast<const uint16_t*>(x), ld_x, reinterpret_cast<const uint16_t*>(weight),
+                          reinterpret_cast<const uint16_t*>(dy), ld_dy, rstd, reinterpret_cast<uint16_t*>(dx), ld_dx,
+                          part, reinterpret_cast<const uint16_t*>(dres), ld_dres, accumulate};
   const int64_t slots = spx_rmsnorm_bwd_slots(rows, H);
-  if (H <= 512)
-    hipLaunchKernelGGL((rmsnorm_bwd_kernel<1, true>), dim3((unsigned)(slots / 4)), dim3(256), 0, st, xp, ld_x,
-                       wp, dyp, ld_dy, rstd, dxp, ld_dx, part, rows, (int)H, drp, ld_dres, accumulate);
-  else if (H <= 4096)
-    hipLaunchKernelGGL((rmsnorm_bwd_kernel<2, false>), dim3((unsigned)slots), dim3(256), 0, st, xp, ld_x, wp,
-                       dyp, ld_dy, rstd, dxp, ld_dx, part, rows, (int)H, drp, ld_dres, accumulate);
-  else
-    hipLaunchKernelGGL((rmsnorm_bwd_kernel<8, false>), dim3((unsigned)slots), dim3(256), 0, st, xp, ld_x, wp,
-                       dyp, ld_dy, rstd, dxp, ld_dx, part, rows, (int)H, drp, ld_dres, accumulate);
+#define SPX_LAUNCH(MAXC, WR, NT)                                                                                    \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, false, NT>), dim3((unsigned)slots), dim3(NT), 0, st, set, set, \
+                     rows, (int)H)
+  SPX_NORM_FORMS(SPX_LAUNCH);
+#undef SPX_LAUNCH
   if (dweight)
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, part, slots, (int)H,
+    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + 31) / 32)), dim3(1024), 0, st, part, slots, (int)H,
                        reinterpret_cast<uint16_t*>(dweight));
   return check_launch(fn);
+}
+
+extern "C" int spx_rmsnorm_pair_bwd_partial(const void* a, int64_t ld_a, const void* weight_a, const void* b,
+                                            int64_t ld_b, const void* weight_b, const void* dy, int64_t ld_dy,
+                                            const void* dres_b, int64_t ld_dres, const float* rstd, void* da,
+                                            void* db, int64_t ld_dx, float* scratch_a, int32_t accumulate_a,
+                                            float* scratch_b, int32_t accumulate_b, int64_t rows, int64_t H,
+                                            void* stream) {
+  SPX_REQUIRE(rows > 0 && H > 0 && H % 8 == 0 && H <= 16384, "rows > 0 and H a multiple of 8, at most 16384");
+  SPX_REQUIRE(ld_a % 8 == 0 && ld_b % 8 == 0 && ld_dy % 8 == 0 && ld_dy >= 2 * H && ld_dres % 8 == 0 &&
+                  ld_dx % 8 == 0, "the row strides must be multiples of 8, that of dy at least 2 H");
+  SPX_REQUIRE(a && weight_a && b && weight_b && dy && rstd && scratch_a && scratch_b, "null buffer");
+  SPX_REQUIRE(!dres_b || db, "a residual gradient needs db");
+  SPX_REQUIRE(al16(a) && al16(weight_a) && al16(b) && al16(weight_b) && al16(dy) && al16(dres_b) && al16(da) &&
+                  al16(db) && al16(scratch_a) && al16(scratch_b), "buffers must be 16-byte aligned");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const uint16_t* dyp = reinterpret_cast<const uint16_t*>(dy);
+  const NormBwdSet one = {reinterpret_cast<const uint16_t*>(a), ld_a, reinterpret_cast<const uint16_t*>(weight_a), dyp,
+                          ld_dy, rstd, reinterpret_cast<uint16_t*>(da), ld_dx, scratch_a, nullptr, 0,
+                          accumulate_a != 0};
+  const NormBwdSet two = {reinterpret_cast<const uint16_t*>(b), ld_b, reinterpret_cast<const uint16_t*>(weight_b),
+                          dyp + H, ld_dy, rstd + rows, reinterpret_cast<uint16_t*>(db), ld_dx, scratch_b,
+                          reinterpret_cast<const uint16_t*>(dres_b), ld_dres, accumulate_b != 0};
+  const int64_t slots = spx_rmsnorm_bwd_slots(rows, H);
+#define SPX_LAUNCH(MAXC, WR, NT)                                                                                      \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, true, NT>), dim3((unsigned)slots, 2), dim3(NT), 0, st, one, two, \
+                     rows, (int)H)
+  SPX_NORM_FORMS(SPX_LAUNCH);
+#undef SPX_LAUNCH
+  return check_launch(__func__);
 }
 
 extern "C" int spx_rmsnorm_bwd(const void* x, int64_t ld_x, const void* weight, const void* dy,
@@ -608,7 +832,7 @@ extern "C" int spx_rmsnorm_dweight(const float* dw_scratch, int64_t slots, int64
   const char* fn = __func__;
   if (!(slots > 0 && H > 0 && H % 8 == 0 && H <= 16384)) return fail_arg(fn, "bad sizes");
   if (!(dw_scratch && dweight && al16(dw_scratch))) return fail_arg(fn, "null or unaligned buffer");
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + 31) / 32)), dim3(256), 0,
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + 31) / 32)), dim3(1024), 0,
                      reinterpret_cast<hipStream_t>(stream), dw_scratch, slots, (int)H,
                      reinterpret_cast<uint16_t*>(dweight));
   return check_launch(fn);
@@ -730,6 +954,52 @@ static int rope_relayout_impl(const char* fn, const void* x, int64_t ld_x, const
     hipLaunchKernelGGL(rope_kernel<false>, dim3(grid), dim3(256), 0, st, xp, ld_x, position_ids, inv_freq, op,
                        ld_out, (int)T, (int)heads, (int)D, (int)rotate, position_offset, (int)tok_head_stride, (int)rot,
                        table_scale);
+  return check_launch(fn);
+}
+
+extern "C" int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_stride, void* k,
+                            int64_t k_head_stride, void* v, int64_t v_head_stride, const int64_t* position_ids,
+                            const float* inv_freq, int64_t T, int32_t hq, int32_t hkv, int32_t D,
+                            int32_t rotary_dim, int32_t inverse, int64_t position_offset, float table_scale,
+                            void* stream) {
+  const char* fn = __func__;
+  SPX_REQ_FN(table_scale > 0.f && table_scale < 1e4f, "the table scale must be positive and finite");
+  SPX_REQ_FN(T > 0 && hq > 0 && hkv > 0 && D > 0 && D % 16 == 0, "T, heads > 0 and D a multiple of 16");
+  SPX_REQ_FN(rotary_dim > 0 && rotary_dim <= D && rotary_dim % 16 == 0,
+             "the rotary dimension must be a multiple of 16 in 16 .. D");
+  const int64_t heads = (int64_t)hq + 2 * (int64_t)hkv;
+  SPX_REQ_FN(ld_tok % 8 == 0 && ld_tok >= heads * D, "bad row stride of the token-major side");
+  SPX_REQ_FN(tok && position_ids && inv_freq && (inverse || (q && k && v)), "null buffer");
+  SPX_REQ_FN(al16(tok) && al16(q) && al16(k) && al16(v), "buffers must be 16-byte aligned");
+  const int64_t win = T * D;
+  SPX_REQ_FN(q_head_stride % 8 == 0 && k_head_stride % 8 == 0 && v_head_stride % 8 == 0 &&
+                 q_head_stride >= win && k_head_stride >= win && v_head_stride >= win,
+             "head strides of the head-major sides must be multiples of 8, at least T * D");
+  const int64_t items = T * heads * (D / 16);
+  SPX_REQ_FN(items < (1ll << 31), "too many elements");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  auto tp = reinterpret_cast<uint16_t*>(tok);
+  auto qp = reinterpret_cast<uint16_t*>(q);
+  auto kp = reinterpret_cast<uint16_t*>(k);
+  auto vp = reinterpret_cast<uint16_t*>(v);
+  // heads per thread: as many as leave every compute unit two workgroups
+#define SPX_LAUNCH(HEADS)                                                                                           \
+  do {                                                                                                              \
+    const int64_t n = T * ((heads + HEADS - 1) / HEADS) * (D / 16);                                                 \
+    const dim3 grid((unsigned)((n + 255) / 256));                                                                   \
+    if (inverse)                                                                                                    \
+      hipLaunchKernelGGL((rope_qkv_kernel<true, HEADS>), grid, dim3(256), 0, st, tp, ld_tok, qp, q_head_stride, kp, \
+                         k_head_stride, vp, v_head_stride, position_ids, inv_freq, (int)T, (int)hq, (int)hkv,       \
+                         (int)D, (int)rotary_dim, position_offset, table_scale);                                    \
+    else                                                                                                            \
+      hipLaunchKernelGGL((rope_qkv_kernel<false, HEADS>), grid, dim3(256), 0, st, tp, ld_tok, qp, q_head_stride,    \
+                         kp, k_head_stride, vp, v_head_stride, position_ids, inv_freq, (int)T, (int)hq, (int)hkv,   \
+                         (int)D, (int)rotary_dim, position_offset, table_scale);                                    \
+  } while (0)
+  if (items >= 4 * 512 * 256) SPX_LAUNCH(4);
+  else if (items >= 2 * 512 * 256) SPX_LAUNCH(2);
+  else SPX_LAUNCH(1);
+#undef SPX_LAUNCH
   return check_launch(fn);
 }
 #undef SPX_REQ_FN

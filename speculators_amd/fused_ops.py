@@ -103,13 +103,15 @@ class GainGrads:
         return dw
 
 
-def _norm_backward(grads, need_dw, x, w, dy, dres, rstd, dx, rows, h):
-    """One launch of the norm's backward; returns the gradient to hand autograd for the gain."""
+def _norm_backward(grads, need_dw, x, w, dy, dres, rstd, dx, rows, h, tgt=None):
+    """One launch of the norm's backward; returns the gradient to hand autograd for the gain.
+    ``tgt``: what ``grads.target`` said already."""
     dev = x.device
     st = _lib.stream_ptr(dev)
     ld_dres = dres.stride(0) if dres is not None else 0
     if need_dw and grads is not None:
-        tgt = grads.target(rows, h, dev)
+        if tgt is None:
+            tgt = grads.target(rows, h, dev)
         if tgt is not None:
             _lib.call("spx_rmsnorm_bwd_partial", x, x.stride(0), w, dy,
                       dy.stride(0), dres, ld_dres, rstd, dx, h,
@@ -193,6 +195,37 @@ def add_rms_norm(a: torch.Tensor, b: torch.Tensor, weight: torch.Tensor, eps: fl
     return _AddRMSNorm.apply(a, b, weight, eps, out)
 
 
+def pair_norm_rows(a2, b2, wa, wb, eps, out, rstd):
+    """Both norms of ``pair_norm_cat`` in one launch: ``out [rows, 2H]``, ``rstd [2, rows]``."""
+    rows, h = a2.shape
+    if rows:
+        _lib.call("spx_rmsnorm_pair_fwd", a2, a2.stride(0), wa, b2, b2.stride(0), wb, out, out.stride(0), rstd,
+                  rows, h, float(eps), _lib.stream_ptr(a2.device))
+
+
+def pair_norm_rows_backward(a2, b2, wa, wb, dy2, dres, rstd, gain_grads, needs):
+    """``(da, db, dwa, dwb)`` of ``pair_norm_rows``; ``needs``: which of ``(a, b, wa, wb)`` want one.
+    One launch where both gains train and share their sums over the uses (``GainGrads``)."""
+    rows, h = a2.shape
+    dev = a2.device
+    dx = [torch.empty(rows, h, device=dev, dtype=torch.bfloat16) if needs[i] else None for i in (0, 1)]
+    tgts = [gain_grads[i].target(rows, h, dev) if needs[2 + i] and gain_grads[i] is not None else None
+            for i in (0, 1)]
+    if tgts[0] is not None and tgts[1] is not None:
+        res = dres if needs[1] else None
+        _lib.call("spx_rmsnorm_pair_bwd_partial", a2, a2.stride(0), wa, b2, b2.stride(0), wb, dy2, dy2.stride(0),
+                  res, res.stride(0) if res is not None else 0, rstd, dx[0], dx[1], h, *tgts[0], *tgts[1], rows, h,
+                  _lib.stream_ptr(dev))
+        return dx[0], dx[1], gain_grads[0].mark(dev), gain_grads[1].mark(dev)
+    dw = [None, None]
+    for i, (x, w) in enumerate(((a2, wa), (b2, wb))):
+        if needs[i] or needs[2 + i]:
+            # (the residual's gradient rides along with b's: dx = rms_norm_bwd(half) + dres)
+            dw[i] = _norm_backward(gain_grads[i], needs[2 + i], x, w, dy2[:, i * h:],
+                                   dres if i == 1 and needs[1] else None, rstd[i], dx[i], rows, h, tgts[i])
+    return dx[0], dx[1], dw[0], dw[1]
+
+
 class _PairNormCat(torch.autograd.Function):
     """``cat([rms_norm(a, wa), rms_norm(b, wb)], -1)`` written straight into the halves of one
     ``[rows, 2H]`` buffer (the input of the first EAGLE3 layer's q/k/v projections,
@@ -215,11 +248,7 @@ class _PairNormCat(torch.autograd.Function):
         rstd = torch.empty(2, rows, device=a.device, dtype=torch.float32)
         ctx.gain_grads = (getattr(wa, "spx_gain_grads", None), getattr(wb, "spx_gain_grads", None))
         wa, wb = wa.contiguous(), wb.contiguous()
-        st = _lib.stream_ptr(a.device)
-        _lib.call("spx_rmsnorm_fwd", a2, a2.stride(0), wa, out, 2 * h,
-                  rstd[0], rows, h, float(eps), st)
-        _lib.call("spx_rmsnorm_fwd", b2, b2.stride(0), wb, out[:, h:], 2 * h,
-                  rstd[1], rows, h, float(eps), st)
+        pair_norm_rows(a2, b2, wa, wb, eps, out, rstd)
         ctx.save_for_backward(a2, b2, wa, wb, rstd)
         ctx.shapes = (a.shape, b.shape)
         cat = out.view(*a.shape[:-1], 2 * h)
@@ -241,17 +270,10 @@ class _PairNormCat(torch.autograd.Function):
             dres = dres.reshape(rows, h).to(torch.bfloat16)
             if dres.stride(1) != 1:
                 dres = dres.contiguous()
-        grads = []
-        for i, (x, w) in enumerate(((a2, wa), (b2, wb))):
-            need_dx, need_dw = ctx.needs_input_grad[i], ctx.needs_input_grad[2 + i]
-            dx = dw = None
-            if need_dx:
-                dx = torch.empty(rows, h, device=x.device, dtype=torch.bfloat16)
-            if need_dx or need_dw:
-                # (the residual's gradient rides along with b's: dx = rms_norm_bwd(half) + dres)
-                dw = _norm_backward(ctx.gain_grads[i], need_dw, x, w, dy2[:, i * h:],
-                                    dres if i == 1 and need_dx else None, rstd[i], dx, rows, h)
-            grads.append((dx.view(ctx.shapes[i]) if dx is not None else None, dw))
+        da, db, dwa, dwb = pair_norm_rows_backward(a2, b2, wa, wb, dy2, dres, rstd, ctx.gain_grads,
+                                                   ctx.needs_input_grad)
+        grads = ((da.view(ctx.shapes[0]) if da is not None else None, dwa),
+                 (db.view(ctx.shapes[1]) if db is not None else None, dwb))
         if dres is not None and not ctx.needs_input_grad[1]:
             raise RuntimeError("the handed-through residual received a gradient but b needs none")
         return grads[0][0], grads[1][0], grads[0][1], grads[1][1], None, None, None

@@ -396,6 +396,31 @@ def linear_staged(x: torch.Tensor, staged, hip: bool = False) -> torch.Tensor:
     return y
 
 
+def _qkv_heads(qkv, position_ids, inv_freq, hq: int, hkv: int, d: int, offset: int, scale: float, kv_out=None):
+    """``qkv [T, (hq + 2 hkv) * d]`` -> rotated q and k, and v, head-major (``kv_out`` as in ``qkv_rope``)."""
+    t, n = qkv.shape
+    q = torch.empty(1, hq, t, d, device=qkv.device, dtype=torch.bfloat16)
+    if kv_out is not None:
+        # [1, Hkv, T, D] windows of the preallocated K / V cache: written in place
+        k, v = kv_out
+    else:
+        kv = torch.empty(2, 1, hkv, t, d, device=qkv.device, dtype=torch.bfloat16)
+        k, v = kv[0], kv[1]
+    _lib.call("spx_rope_qkv", qkv, n, q, t * d, k, k.stride(1), v, v.stride(1), position_ids, inv_freq, t, hq, hkv, d,
+              2 * inv_freq.numel(), 0, offset, scale, _lib.stream_ptr(qkv.device))
+    return q, k, v
+
+
+def _qkv_tokens(dqkv, grads, position_ids, inv_freq, hq: int, hkv: int, d: int, offset: int, scale: float):
+    """The way back of ``_qkv_heads`` for the gradients ``grads`` (None: zeros) into ``dqkv``."""
+    t, n = dqkv.shape
+    dq, dk, dv = grads
+    win = t * d
+    _lib.call("spx_rope_qkv", dqkv, n, dq, dq.stride(1) if dq is not None else win,
+              dk, dk.stride(1) if dk is not None else win, dv, dv.stride(1) if dv is not None else win, position_ids,
+              inv_freq, t, hq, hkv, d, 2 * inv_freq.numel(), 1, offset, scale, _lib.stream_ptr(dqkv.device))
+
+
 class _QKVRope(torch.autograd.Function):
     """q/k/v projections of one input as ONE GEMM against the staged concatenation of the three
     weights, followed by the rotary embedding + head-major relayout of each part.  The backward
@@ -413,51 +438,32 @@ class _QKVRope(torch.autograd.Function):
         x2 = x.reshape(t, x.shape[-1])
         qkv = _project(x2, staged)
         n = qkv.shape[1]
-        st = _lib.stream_ptr(x.device)
         scale = FO.table_scale_of(inv_freq)
-        outs, col = [], 0
-        for idx, (heads, rotate) in enumerate(((hq, 1), (hkv, 1), (hkv, 0))):
-            if idx and kv_out is not None:
-                # a [1, Hkv, T, D] window of the preallocated K / V cache: written in place
-                out = kv_out[idx - 1]
-                head_stride = out.stride(1)
-            else:
-                out = torch.empty(1, heads, t, d, device=x.device, dtype=torch.bfloat16)
-                head_stride = 0
-            part = qkv[:, col:]
-            FO.rope_call(part, n, d, position_ids, inv_freq, out, head_stride, t, heads, d,
-                         rotate, 0, offset, scale, st)
-            outs.append(out)
-            col += heads * d
+        outs = _qkv_heads(qkv, position_ids, inv_freq, hq, hkv, d, offset, scale, kv_out)
         ctx.save_for_backward(x2, wcat, position_ids, inv_freq)
         ctx.meta = (x.shape, hq, hkv, d, offset, n, staged, scale)
         ctx.slot = staged.take(x2) if ctx.needs_input_grad[1] else -1
         ctx.set_materialize_grads(False)
-        return tuple(outs)
+        return outs
 
     @staticmethod
     def backward(ctx, dq, dk, dv):
         x2, wcat, position_ids, inv_freq = ctx.saved_tensors
         shape, hq, hkv, d, offset, n, staged, scale = ctx.meta
         t = x2.shape[0]
-        st = _lib.stream_ptr(x2.device)
         dqkv = staged.dy_slot(ctx.slot, t) if ctx.needs_input_grad[1] else None
         if dqkv is None:
             dqkv = torch.empty(t, n, device=x2.device, dtype=torch.bfloat16)
-        col = 0
-        for g, heads, rotate in ((dq, hq, 1), (dk, hkv, 1), (dv, hkv, 0)):
-            part = dqkv[:, col:]
-            if g is None:
-                dqkv[:, col:col + heads * d].zero_()
-            else:
+        grads = []
+        for g in (dq, dk, dv):
+            if g is not None:
                 g = g.to(torch.bfloat16)
                 # a window of a longer gradient tensor is read in place through its head stride
                 if not (g.stride(3) == 1 and g.stride(2) == d and g.stride(1) % 8 == 0
                         and g.stride(1) >= t * d and g.data_ptr() % 16 == 0):
                     g = g.contiguous()
-                FO.rope_call(g, g.stride(1), d, position_ids, inv_freq, part, n, t, heads, d,
-                             rotate, 1, offset, scale, st)
-            col += heads * d
+            grads.append(g)
+        _qkv_tokens(dqkv, grads, position_ids, inv_freq, hq, hkv, d, offset, scale)
         dx = dw = None
         if ctx.needs_input_grad[0]:
             dx = _project_back(dqkv, staged).view(shape)

@@ -347,3 +347,56 @@ def test_transposed_copy_of_a_matrix_or_a_stack(shape):
     w = torch.randn(*shape, generator=g).bfloat16().cuda()
     got = transposed_copy(w)
     assert got.is_contiguous() and torch.equal(got, w.transpose(-1, -2).contiguous())
+
+
+@pytest.mark.parametrize("rows,h", [(1100, 2048), (70, 2056), (9, 4104), (1500, 8192), (33, 16384), (8200, 128), (3, 512)])
+def test_norm_backward_at_every_row_width(rows, h):
+    """Both gradients, where the threads a row is spread over change and at more rows than slots."""
+    from speculators_amd.fused_ops import rms_norm
+
+    g = torch.Generator().manual_seed(rows * h)
+    x = (torch.randn(1, rows, h, generator=g) * 2).bfloat16()
+    w = (1 + 0.2 * torch.randn(h, generator=g)).bfloat16()
+    go = torch.randn(1, rows, h, generator=g).bfloat16()
+    xg, wg = x.cuda().requires_grad_(True), w.cuda().requires_grad_(True)
+    rms_norm(xg, wg, 1e-5).backward(go.cuda())
+    xr, wr = x.float().requires_grad_(True), w.float().requires_grad_(True)
+    OE.rms_norm(xr, wr, 1e-5).backward(go.float())
+    _close(xg.grad, xr.grad)
+    _close(wg.grad, wr.grad)
+
+
+@pytest.mark.parametrize("t,hq,hkv,d,rot", [(1, 1, 1, 64, 64), (77, 5, 2, 128, 128), (700, 16, 8, 128, 128),
+                                            (1500, 32, 9, 64, 64), (900, 9, 5, 128, 64), (1100, 24, 3, 128, 128)])
+def test_rope_qkv_is_the_three_relayouts(t, hq, hkv, d, rot):
+    """One launch for q, k and v (1, 2 and 4 heads a thread, head counts that leave a remainder) gives the bits of
+    the relayout kernel on each part, both ways, k and v in windows of a longer cache."""
+    from speculators_amd import _lib
+    from speculators_amd.fused_ops import rope_call, rope_inv_freq
+
+    g = torch.Generator().manual_seed(t)
+    n = (hq + 2 * hkv) * d
+    qkv = torch.randn(t, n, generator=g).bfloat16().cuda()
+    pos = torch.randint(0, 9000, (t,), generator=g).cuda()
+    inv = rope_inv_freq(rot, 500000.0, "cuda")
+    st = _lib.stream_ptr(qkv.device)
+    cache = torch.zeros(2, hkv, 3 * t, d, device="cuda", dtype=torch.bfloat16)
+    k, v = cache[0][:, t:2 * t], cache[1][:, t:2 * t]
+    q = torch.empty(hq, t, d, device="cuda", dtype=torch.bfloat16)
+    hs = 3 * t * d
+    _lib.call("spx_rope_qkv", qkv, n, q, t * d, k, hs, v, hs, pos, inv, t, hq, hkv, d, rot, 0, 2, 1.0, st)
+    parts = [(q, hq, 1), (k, hkv, 1), (v, hkv, 0)]
+    back, col = torch.empty_like(qkv), 0
+    for got, heads, rotate in parts:
+        want = torch.empty(heads, t, d, device="cuda", dtype=torch.bfloat16)
+        rope_call(qkv[:, col:], n, d, pos, inv, want, 0, t, heads, d, rotate, 0, 2, 1.0, st)
+        assert torch.equal(got, want)
+        rope_call(want, 0, d, pos, inv, back[:, col:], n, t, heads, d, rotate, 1, 2, 1.0, st)
+        col += heads * d
+    assert not cache[:, :, :t].any() and not cache[:, :, 2 * t:].any()
+    got = torch.empty_like(qkv)
+    _lib.call("spx_rope_qkv", got, n, q, t * d, k, hs, v, hs, pos, inv, t, hq, hkv, d, rot, 1, 2, 1.0, st)
+    assert torch.equal(got, back)
+    _lib.call("spx_rope_qkv", got, n, q, t * d, None, hs, v, hs, pos, inv, t, hq, hkv, d, rot, 1, 2, 1.0, st)
+    back[:, hq * d:(hq + hkv) * d] = 0
+    assert torch.equal(got, back)
