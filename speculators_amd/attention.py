@@ -141,6 +141,63 @@ class _CacheGrads:
         self.task, self.dk, self.dv, self.low = -1, None, None, 0
 
 
+def ttt_forward_into(q, k, v, mask: TTTMask, scaling: float, out) -> torch.Tensor:
+    """The forward kernel into ``out`` (``T * Hq * D`` contiguous bf16 elements); returns the row statistics."""
+    _, hq, t, d = q.shape
+    hkv = k.shape[1]
+    dev = q.device
+    lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
+    nbytes = _workspace_bytes(t, hq, hkv, d, False)
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    _lib.call("spx_ttt_attn_fwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), mask.row_lo, t, mask.ttt_step, hq,
+              hkv, d, float(scaling), out, lse, ws, nbytes, _lib.stream_ptr(dev))
+    return lse
+
+
+def _ttt_backward_cached(g: _CacheGrads, q, k, v, out, dout, lse, mask: TTTMask, n: int, scaling: float):
+    """``(dq, dk, dv)`` of the step whose keys are the last of ``n``: dk / dv over all ``n`` steps' keys, in the
+    buffers the pass shares (see ``_TTTAttentionCached``)."""
+    _, hq, t, d = q.shape
+    hkv = k.shape[1]
+    dev = q.device
+    dq = torch.empty_like(q)
+    task = torch._C._current_graph_task_id()
+    shared = task >= 0
+    if shared and g.task == task:
+        if n > g.low:
+            raise RuntimeError("the attention node of a later TTT step ran after an earlier step's "
+                               "in one backward pass")
+        entry = "spx_ttt_attn_bwd_accumulate"
+        dk, dv = g.dk[:, :, :n * t], g.dv[:, :, :n * t]
+    else:
+        entry = "spx_ttt_attn_bwd"
+        dk = torch.empty(1, hkv, n * t, d, device=dev, dtype=torch.bfloat16)
+        dv = torch.empty(1, hkv, n * t, d, device=dev, dtype=torch.bfloat16)
+        if shared:
+            g.task, g.dk, g.dv = task, dk, dv
+    nbytes = _workspace_bytes(t, hq, hkv, d, True)
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    _lib.call(entry, q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo, t, mask.ttt_step,
+              hq, hkv, d, scaling, dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1), ws, nbytes,
+              _lib.stream_ptr(dev))
+    return dq, dk, dv
+
+
+def ttt_backward_shared(g: _CacheGrads, q, k, v, out, dout, lse, mask: TTTMask, n: int, scaling: float):
+    """``(dq, dk, dv)`` of one step inside a backward pass, dk / dv of the step's OWN keys: complete, because
+    the nodes of all later steps have run."""
+    if torch._C._current_graph_task_id() < 0:
+        raise RuntimeError("the backward of a layer step runs inside a backward pass of autograd only")
+    t = q.shape[2]
+    dq, dk, dv = _ttt_backward_cached(g, q, k, v, out, dout, lse, mask, n, scaling)
+    g.low = n
+    lo = (n - 1) * t
+    dk, dv = dk[:, :, lo:], dv[:, :, lo:]
+    if n == 1:  # the first step's node is the last to run: the pass is done with the buffers
+        g.task, g.dk, g.dv = -1, None, None
+    return dq, dk, dv
+
+
 class _TTTAttentionCached(torch.autograd.Function):
     """TTT attention over a ``TTTKVCache``: the per-step key / value tensors (windows of the
     cache, already written) are the differentiable inputs, the kernels read the cache in place.
@@ -163,12 +220,7 @@ class _TTTAttentionCached(torch.autograd.Function):
             out = out.view(1, t, hq, d)
         else:
             out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
-        lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_fwd", q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), mask.row_lo, t, mask.ttt_step, hq, hkv, d,
-                  float(scaling), out, lse, ws, ws.numel(),
-                  _lib.stream_ptr(dev))
+        lse = ttt_forward_into(q, k, v, mask, scaling, out)
         ctx.save_for_backward(q, out, lse)
         ctx.kv = (k, v)  # windows of the cache: later steps only write rows beyond them
         ctx.mask, ctx.scaling, ctx.n_parts = mask, float(scaling), n_parts
@@ -180,32 +232,11 @@ class _TTTAttentionCached(torch.autograd.Function):
         q, out, lse = ctx.saved_tensors
         k, v = ctx.kv
         mask, n = ctx.mask, ctx.n_parts
-        _, hq, t, d = q.shape
-        hkv = k.shape[1]
-        dev = q.device
+        t = q.shape[2]
         dout = dout.to(torch.bfloat16).contiguous()
-        dq = torch.empty_like(q)
         g = ctx.grads
-        task = torch._C._current_graph_task_id()
-        shared = task >= 0
-        if shared and g.task == task:
-            if n > g.low:
-                raise RuntimeError("the attention node of a later TTT step ran after an earlier step's "
-                                   "in one backward pass")
-            entry = "spx_ttt_attn_bwd_accumulate"
-            dk, dv = g.dk[:, :, :n * t], g.dv[:, :, :n * t]
-        else:
-            entry = "spx_ttt_attn_bwd"
-            dk = torch.empty(1, hkv, n * t, d, device=dev, dtype=torch.bfloat16)
-            dv = torch.empty(1, hkv, n * t, d, device=dev, dtype=torch.bfloat16)
-            if shared:
-                g.task, g.dk, g.dv = task, dk, dv
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call(entry, q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), out, dout, lse,
-                  mask.row_lo, t, mask.ttt_step, hq, hkv, d, ctx.scaling,
-                  dq, dq.stride(1), dk, dk.stride(1), dv,
-                  dv.stride(1), ws, ws.numel(), _lib.stream_ptr(dev))
+        shared = torch._C._current_graph_task_id() >= 0
+        dq, dk, dv = _ttt_backward_cached(g, q, k, v, out, dout, lse, mask, n, ctx.scaling)
         if not shared:  # outside a backward pass of the engine: every step's window, to be summed by the caller
             dks = [dk[:, :, i * t:(i + 1) * t] for i in range(n)]
             dvs = [dv[:, :, i * t:(i + 1) * t] for i in range(n)]

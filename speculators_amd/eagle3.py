@@ -26,6 +26,7 @@ from torch import nn
 from . import attention as A
 from . import fused_ops as FO
 from . import gemm
+from . import layer as LY
 from . import losses as L
 from . import metrics as MT
 from .weights import WeightStager, compute_input
@@ -175,11 +176,43 @@ class DecoderLayer(nn.Module):
         if self.first:
             self.hidden_norm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, stager)
 
-    def forward(self, x, position_ids, pos_offset, inv_freq, cache, mask, next_norm=None):
+    def _step(self, position_ids, pos_offset, inv_freq, cache, mask, next_norm, t, device):
+        """The layer's next TTT step as one node (``layer.LayerStep``), or None where the layer is put
+        together from its parts: per-head norms, another attention function or head size, the normalised
+        hidden state as residual, or a graph in which some projection does not train."""
+        att, cfg = self.self_attn, self.cfg
+        if (next_norm is None or att.qk_norm or att.attn_fn is not A.ttt_hip_attention_forward
+                or att.d not in A.KERNEL_HEAD_DIMS or not cache.get("steps")
+                or (self.first and cfg.norm_before_residual)):
+            return None
+        W = self._stager.get
+        ws = (self._wqkv(), W(att.o_proj.weight), W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight),
+              W(self.mlp.down_proj.weight))
+        if torch.is_grad_enabled() and not all(w.trainable for w in ws):
+            return None
+        kvc = cache.get("kv")
+        if kvc is None:
+            kvc = cache["kv"] = A.TTTKVCache(att.hkv, t, att.d, cache["steps"], device)
+        return LY.LayerStep(self.first, *ws, (cfg.rms_norm_eps, self.post_attention_layernorm.eps, next_norm.eps),
+                            (att.hq, att.hkv, att.d), att.scaling, pos_offset, position_ids, inv_freq, kvc, mask)
+
+    def _wqkv(self):
+        att = self.self_attn
+        return self._stager.get(att.q_proj.weight, att.k_proj.weight, att.v_proj.weight)
+
+    def forward(self, x, position_ids, pos_offset, inv_freq, cache, mask, next_norm=None, next_layer=None):
         """``x``: the hidden state, or for the first layer the pair ``(embeds, hidden)`` (their
         concatenation is what the reference passes).  With ``next_norm`` (the RMSNorm that
         consumes this layer's output) the result is ``(out, next_norm(out))``: the last
-        residual add is fused into that norm."""
+        residual add is fused into that norm.  ``next_layer``: the layer that reads it, if one does."""
+        if self.first or isinstance(x, _Prenormed):
+            one, two = x
+            step = self._step(position_ids, pos_offset, inv_freq, cache, mask, next_norm, two.shape[1], two.device)
+            if step is not None and one.dtype == two.dtype == torch.bfloat16:
+                step.take_slots(two.shape[1], None if next_layer is None or next_layer.self_attn.qk_norm
+                                else next_layer._wqkv())
+                gains = (self.input_layernorm.gain, self.hidden_norm.gain) if self.first else (None, None)
+                return LY.run(step, one, two, *gains, self.post_attention_layernorm.gain, next_norm.gain)
         if self.first:
             embeds, hidden = x
             eps = self.cfg.rms_norm_eps
@@ -367,7 +400,8 @@ class Eagle3DraftModel(nn.Module):
                 # the norm that reads this layer's output: the next layer's input norm, or the
                 # final norm -- the layer fuses its last residual add into it
                 nxt = self.norm if li == last else self.layers[li + 1].input_layernorm
-                y, normed = layer(y, position_ids, step, inv_freq, caches[li], mask, next_norm=nxt)
+                y, normed = layer(y, position_ids, step, inv_freq, caches[li], mask, next_norm=nxt,
+                                  next_layer=None if li == last else self.layers[li + 1])
                 if li != last:
                     y = _Prenormed(y, normed)
             hidden = normed if cfg.norm_output else y

@@ -400,3 +400,42 @@ def test_rope_qkv_is_the_three_relayouts(t, hq, hkv, d, rot):
     _lib.call("spx_rope_qkv", got, n, q, t * d, None, hs, v, hs, pos, inv, t, hq, hkv, d, rot, 1, 2, 1.0, st)
     back[:, hq * d:(hq + hkv) * d] = 0
     assert torch.equal(got, back)
+
+
+@pytest.mark.parametrize("layers,norm_output,fp32", [(1, False, False), (2, True, True)])
+def test_layer_step_node_is_the_layer_from_its_parts(layers, norm_output, fp32, monkeypatch):
+    from speculators_amd import eagle3 as E
+
+    cfg = E.Eagle3Config(hidden_size=256, num_attention_heads=4, num_key_value_heads=2, head_dim=64,
+                         intermediate_size=320, vocab_size=512, draft_vocab_size=512, num_hidden_layers=layers,
+                         norm_output=norm_output, sliding_window=40, sliding_layers=(layers - 1,))
+    torch.manual_seed(3)
+    model = E.Eagle3DraftModel(cfg).cuda()
+    if not fp32:
+        model = model.bfloat16()
+    t = 150
+    g = torch.Generator().manual_seed(4)
+    batch = dict(hidden_states=torch.randn(1, t, 768, generator=g).bfloat16().cuda(),
+                 input_ids=torch.randint(0, 512, (1, t), generator=g).cuda(),
+                 document_ids=torch.arange(t).div(60, rounding_mode="floor").view(1, t).cuda(),
+                 loss_mask=(torch.rand(1, t, generator=g) < 0.7).cuda(),
+                 verifier_last_hidden_states=torch.randn(1, t, 256, generator=g).bfloat16().cuda(), ttt_steps=3)
+
+    def step():
+        model.zero_grad()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            tokens, loss, _ = model(**batch)
+        loss.backward()
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            val = model(**batch)[1]
+        return tokens, loss, val, {n: p.grad for n, p in model.named_parameters() if p.grad is not None}
+
+    got = step()
+    monkeypatch.setattr(E.DecoderLayer, "_step", lambda self, *a: None)
+    want = step()
+    assert all(torch.equal(a, b) for a, b in zip(got[0], want[0], strict=True))
+    assert got[1].item() == want[1].item() and got[2].item() == want[2].item()
+    assert got[3].keys() == want[3].keys() and len(want[3]) >= 10 * layers
+    for n, a in want[3].items():
+        # (the second layer's q/k/v gradient is one product over the steps instead of one each)
+        _close(got[3][n], a.cpu(), rel=1e-2 if layers > 1 else 0.0)
