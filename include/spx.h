@@ -272,6 +272,23 @@ int spx_ttt_step_mean(const float* loss, const void* mask, int mask_kind, int64_
                       float weight, const int32_t* counts, float* out, float* row_weight,
                       void* stream);
 
+/* Either of the two above (counts NULL: as spx_ttt_step_reduce) together with the term's place in the loss:
+ * out has 8 elements, out[6] = factor * out[0], out[7] = 1, and *total_out = out[6] (+ *total_in, may be NULL). */
+int spx_ttt_step_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target,
+                       const void* mask, int mask_kind, void* prev_correct, int prev_kind, int64_t rows,
+                       float weight, const int32_t* counts, float factor, const float* total_in,
+                       float* total_out, float* out, float* row_weight, void* stream);
+
+/* spx_pack_row_map for a row mask of any element kind (live: not zero); zero3 (int32[3], may be NULL) is
+ * cleared: the counts of the loss pass that follows. */
+int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
+                     int32_t* zero3, void* stream);
+
+/* Draft tokens: out[i] = known[i] for i < n (int32 arg-maxes of a loss pass, widened), out[n + j] = the first
+ * index of the maximum of row j < tail of rows[tail, vocab] (bf16 / f32, row stride ld). */
+int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail, int64_t vocab,
+                   int dtype, int64_t* out, void* stream);
+
 /* Weighted masked mean and per-slot acceptance counts of a DFlash block batch:
  *   out[0] = sum_r loss[r] m_r w_r / (sum m + 1e-5),  out[1] = sum m
  *   correct[s], total[s]  (s < block_size): matches / rows with m_r != 0 at
@@ -667,6 +684,11 @@ int spx_unpack_rows(const void* packed, int64_t ld_packed, const int32_t* row_ma
 int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, const int32_t* row_map,
                            const float* row_scale, int64_t rows, int64_t total_rows,
                            int64_t cols, void* out, int64_t ld_out, void* stream);
+
+/* The same with row_scale[r] * (*scale * factor); scale: one f32 on the device (NULL: 1 and no factor). */
+int spx_unpack_rows_graded(const void* packed, int64_t ld_packed, const int32_t* row_map,
+                           const float* row_scale, const float* scale, float factor, int64_t rows,
+                           int64_t total_rows, int64_t cols, void* out, int64_t ld_out, void* stream);
 
 /* c[M, N] (+)= a[T, M]^T * b[T, N], bf16 inputs, fp32 accumulation, bf16 output:
  * the weight-gradient product of the backward of torch.nn.Linear (dW = dY^T X)

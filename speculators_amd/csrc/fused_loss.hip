@@ -62,16 +62,6 @@ __device__ __forceinline__ float log_mix(float la, float lb) {
   return mx + fast_log2(s) * kLn2 - kLn2;
 }
 
-// ---- mask element access ---------------------------------------------------
-__device__ __forceinline__ float mask_value(const void* p, int kind, int64_t i) {
-  switch (kind) {
-    case SPX_KIND_U8: return (float)reinterpret_cast<const uint8_t*>(p)[i];
-    case SPX_KIND_I32: return (float)reinterpret_cast<const int32_t*>(p)[i];
-    case SPX_KIND_I64: return (float)reinterpret_cast<const int64_t*>(p)[i];
-    case SPX_KIND_F32: return reinterpret_cast<const float*>(p)[i];
-    default: return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p)[i]);
-  }
-}
 __device__ __forceinline__ void store_flag(void* p, int kind, int64_t i, bool v) {
   switch (kind) {
     case SPX_KIND_U8: reinterpret_cast<uint8_t*>(p)[i] = v ? 1 : 0; break;
@@ -902,7 +892,8 @@ __global__ __launch_bounds__(kReduceThreads) void ttt_step_reduce_kernel(
     const float* __restrict__ loss, const int32_t* __restrict__ pred,
     const int32_t* __restrict__ tgt, const void* __restrict__ mask, int mask_kind,
     void* prev, int prev_kind, int64_t rows, float weight, float* __restrict__ out,
-    float* __restrict__ row_weight, const int32_t* __restrict__ counts) {
+    float* __restrict__ row_weight, const int32_t* __restrict__ counts,
+    float factor, const float* __restrict__ total_in, float* __restrict__ total_out) {
   __shared__ float fl[kReduceThreads / 64];
   __shared__ int il[kReduceThreads / 64];
   float lsum = 0.f, msum = 0.f;
@@ -939,12 +930,61 @@ __global__ __launch_bounds__(kReduceThreads) void ttt_step_reduce_kernel(
     out[3] = (float)correct;
     out[4] = (prev || counts) ? (float)cond_total : (float)rows;
     out[5] = msum;
+    if (total_out) {  // the term in the loss: what a handful of one-element kernels did
+      const float part = lsum * inv * factor;
+      out[6] = part;
+      out[7] = 1.f;
+      *total_out = total_in ? *total_in + part : part;
+    }
   }
   if (row_weight) {
     for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
       float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
       row_weight[r] = m * inv;
     }
+  }
+}
+
+// The rows a mask leaves, in order, and three zeroed counters for the loss pass behind it.
+__global__ __launch_bounds__(1024) void mask_row_map_kernel(const void* __restrict__ mask, int mask_kind, int rows,
+                                                            int32_t* __restrict__ row_map,
+                                                            int32_t* __restrict__ count, int32_t* __restrict__ zero3) {
+  if (zero3 && threadIdx.x < 3) zero3[threadIdx.x] = 0;
+  pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, rows, row_map, count);
+}
+
+// Draft tokens (int64): the known arg-maxes of the first n rows widened, the arg-max (first index of the
+// maximum) of the rows behind them, one workgroup each.  One launch for a conversion, an arg-max pass over few
+// rows, another conversion and a concatenation.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kLossThreads) void row_tokens_kernel(const int32_t* __restrict__ known, int n,
+                                                                  const T* __restrict__ rows, int64_t ld,
+                                                                  int64_t vocab, int tail, int64_t* __restrict__ out) {
+  if ((int)blockIdx.x >= tail) {
+    const int i = ((int)blockIdx.x - tail) * kLossThreads + threadIdx.x;
+    if (i < n) out[i] = known[i];
+    return;
+  }
+  const T* row = rows + (int64_t)blockIdx.x * ld;
+  float best = -INFINITY;
+  int at = 0x7fffffff;
+  for (int64_t base = (int64_t)threadIdx.x * 8; base < vocab; base += kLossThreads * 8) {
+    float x[8];
+    load8<T, VEC>(row, base, vocab, x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (x[i] > best && base + i < vocab) { best = x[i]; at = (int)(base + i); }
+  }
+  auto take = [&](float b, int a) { if (b > best || (b == best && a < at)) { best = b; at = a; } };
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) take(__shfl_xor(best, m, 64), __shfl_xor(at, m, 64));
+  __shared__ float bl[kLossWaves];
+  __shared__ int al[kLossWaves];
+  if ((threadIdx.x & 63) == 0) { bl[threadIdx.x >> 6] = best; al[threadIdx.x >> 6] = at; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kLossWaves; ++w) take(bl[w], al[w]);
+    out[n + (int64_t)blockIdx.x] = at;
   }
 }
 
@@ -1267,7 +1307,8 @@ extern "C" int spx_ttt_step_reduce(const float* loss, const int32_t* argmax_draf
   SPX_REQUIRE(!prev_correct || kind_ok(prev_kind), "unknown prev_correct element kind");
   hipLaunchKernelGGL(ttt_step_reduce_kernel, dim3(1), dim3(kReduceThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), loss, argmax_draft, argmax_target, mask,
-                     mask_kind, prev_correct, prev_kind, rows, weight, out, row_weight, nullptr);
+                     mask_kind, prev_correct, prev_kind, rows, weight, out, row_weight, nullptr, 1.f, nullptr,
+                     nullptr);
   return check_launch(__func__);
 }
 
@@ -1279,7 +1320,48 @@ extern "C" int spx_ttt_step_mean(const float* loss, const void* mask, int mask_k
   SPX_REQUIRE(!mask || kind_ok(mask_kind), "unknown mask element kind");
   hipLaunchKernelGGL(ttt_step_reduce_kernel, dim3(1), dim3(kReduceThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), loss, nullptr, nullptr, mask, mask_kind,
-                     nullptr, 0, rows, weight, out, row_weight, counts);
+                     nullptr, 0, rows, weight, out, row_weight, counts, 1.f, nullptr, nullptr);
+  return check_launch(__func__);
+}
+
+extern "C" int spx_ttt_step_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target,
+                                  const void* mask, int mask_kind, void* prev_correct, int prev_kind, int64_t rows,
+                                  float weight, const int32_t* counts, float factor, const float* total_in,
+                                  float* total_out, float* out, float* row_weight, void* stream) {
+  SPX_REQUIRE(rows >= 0 && rows < (1ll << 24), "0 <= rows < 2^24");
+  SPX_REQUIRE(loss && out && total_out && (counts || (argmax_draft && argmax_target)), "null buffer");
+  SPX_REQUIRE(!mask || kind_ok(mask_kind), "unknown mask element kind");
+  SPX_REQUIRE(!prev_correct || kind_ok(prev_kind), "unknown prev_correct element kind");
+  hipLaunchKernelGGL(ttt_step_reduce_kernel, dim3(1), dim3(kReduceThreads), 0,
+                     reinterpret_cast<hipStream_t>(stream), loss, argmax_draft, argmax_target, mask, mask_kind,
+                     prev_correct, prev_kind, rows, weight, out, row_weight, counts, factor, total_in, total_out);
+  return check_launch(__func__);
+}
+
+extern "C" int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
+                                int32_t* zero3, void* stream) {
+  SPX_REQUIRE(rows > 0 && rows < (1ll << 31), "rows out of range");
+  SPX_REQUIRE(mask && row_map && count && kind_ok(mask_kind), "null buffer or unknown mask element kind");
+  hipLaunchKernelGGL(mask_row_map_kernel, dim3(1), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), mask,
+                     mask_kind, (int)rows, row_map, count, zero3);
+  return check_launch(__func__);
+}
+
+extern "C" int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail,
+                              int64_t vocab, int dtype, int64_t* out, void* stream) {
+  SPX_REQUIRE(dtype == SPX_DTYPE_BF16 || dtype == SPX_DTYPE_F32, "dtype must be bf16 or f32");
+  SPX_REQUIRE(n >= 0 && tail >= 0 && n + tail < (1ll << 31) && vocab > 0 && vocab < (1ll << 31), "sizes out of range");
+  if (n + tail == 0) return SPX_OK;
+  SPX_REQUIRE(out && (n == 0 || known) && (tail == 0 || (rows && ld >= vocab)), "null buffer or short row stride");
+  const dim3 grid((unsigned)(tail + (n + kLossThreads - 1) / kLossThreads));
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const bool vec = aligned16(rows) && ld % (dtype == SPX_DTYPE_BF16 ? 8 : 4) == 0;
+#define SPX_TOKENS(T, VEC)                                                                                    \
+  hipLaunchKernelGGL((row_tokens_kernel<T, VEC>), grid, dim3(kLossThreads), 0, st, known, (int)n,            \
+                     reinterpret_cast<const T*>(rows), ld, vocab, (int)tail, out)
+  if (dtype == SPX_DTYPE_BF16) { if (vec) SPX_TOKENS(uint16_t, true); else SPX_TOKENS(uint16_t, false); }
+  else { if (vec) SPX_TOKENS(float, true); else SPX_TOKENS(float, false); }
+#undef SPX_TOKENS
   return check_launch(__func__);
 }
 

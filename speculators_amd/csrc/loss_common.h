@@ -3,6 +3,7 @@
 #pragma once
 
 #include "spx_common.h"
+#include "../../include/spx.h"
 
 namespace spx {
 
@@ -92,6 +93,48 @@ __device__ __forceinline__ void store8(T* row, int64_t base, int64_t n, const fl
 
 __host__ __device__ __forceinline__ bool ptr_aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+}
+
+// ---- mask element access ---------------------------------------------------
+__device__ __forceinline__ float mask_value(const void* p, int kind, int64_t i) {
+  switch (kind) {
+    case SPX_KIND_U8: return (float)reinterpret_cast<const uint8_t*>(p)[i];
+    case SPX_KIND_I32: return (float)reinterpret_cast<const int32_t*>(p)[i];
+    case SPX_KIND_I64: return (float)reinterpret_cast<const int64_t*>(p)[i];
+    case SPX_KIND_F32: return reinterpret_cast<const float*>(p)[i];
+    default: return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p)[i]);
+  }
+}
+
+// row_map[r] = number of live rows before r if live(r), else -1; *count = number of live rows.  One workgroup
+// of 1024 threads, rows in order.
+template <typename Live>
+__device__ __forceinline__ void pack_row_map(Live live_at, int rows, int32_t* __restrict__ row_map,
+                                             int32_t* __restrict__ count) {
+  __shared__ int wave_tot[16];
+  __shared__ int base_s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) base_s = 0;
+  __syncthreads();
+  for (int r0 = 0; r0 < rows; r0 += 1024) {
+    const int r = r0 + tid;
+    const bool live = r < rows && live_at(r);
+    const unsigned long long m = __ballot(live);
+    const int before = __popcll(m & ((1ull << lane) - 1ull));
+    if (lane == 0) wave_tot[wave] = __popcll(m);
+    __syncthreads();
+    int off = base_s;
+    for (int w = 0; w < wave; ++w) off += wave_tot[w];
+    if (r < rows) row_map[r] = live ? off + before : -1;
+    __syncthreads();
+    if (tid == 0) {
+      int t = 0;
+      for (int w = 0; w < 16; ++w) t += wave_tot[w];
+      base_s += t;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) *count = base_s;
 }
 
 }  // namespace spx

@@ -357,7 +357,9 @@ class Eagle3DraftModel(nn.Module):
             x = torch.cat([n(c) for n, c in zip(self.fc_norm, chunks, strict=True)], dim=-1)
         hidden = self._linear(x, self.fc.weight)
 
-        original_ids = input_ids.detach().clone()
+        # the ids of step j are the given ones shifted by j, zeros behind them: windows of one buffer
+        ids = torch.zeros(1, t + ttt_steps, device=device, dtype=input_ids.dtype)
+        ids[:, :t].copy_(input_ids.detach())
         return_loss = verifier_last_hidden_states is not None or verifier_logits is not None
         if return_loss:
             with torch.no_grad():
@@ -370,7 +372,7 @@ class Eagle3DraftModel(nn.Module):
                     # head product's epilogue and never sees the rows (metrics.VerifierHead)
                     targets = MT.VerifierHead(self.verifier_norm(verifier_last_hidden_states),
                                               self._stager.get(self.verifier_lm_head.weight).w)
-            loss = torch.zeros((), device=device)
+            loss = None
             prev_correct = (loss_mask.clone() if loss_mask is not None
                             else torch.ones(1, t, device=device, dtype=torch.bool))
             metrics: dict = {}
@@ -389,7 +391,7 @@ class Eagle3DraftModel(nn.Module):
                 table = self.embed_tokens.weight
                 if not table.requires_grad:
                     table = self._stager.get(table).w  # frozen: its bf16 copy is made once and kept
-                embeds = F.embedding(input_ids, table)
+                embeds = F.embedding(ids[:, step:step + t], table)
             y = (embeds.to(hidden.dtype), hidden)
             normed = None
             last = len(self.layers) - 1
@@ -414,26 +416,20 @@ class Eagle3DraftModel(nn.Module):
             if return_loss:
                 # head + loss as one autograd node while the head is frozen (see metrics.Head)
                 lg = MT.Head(normed, head.w, head.wt) if fuse else logits
-                s_loss, s_metrics, pred = MT.compute_metrics(
-                    lg, targets, loss_mask, prev_correct, step, ttt_step_loss_decay,
-                    loss_config=loss_config, target_stats_cache=stats_cache, return_pred=True)
-                if fuse:
-                    logits = lg.logits
-                loss = loss + s_loss
-                metrics.update(s_metrics)
                 # draft tokens: the loss kernel's arg-max for the aligned rows, plus the
                 # last `step` rows (which have no target) on their own
-                pred = pred.to(torch.int64)
-                if step:
-                    pred = torch.cat([pred, MT.argmax_rows(logits.detach()[0, t - step:])])
-                draft_tokens.append(pred.view(1, t))
+                loss, s_metrics, tokens = MT.compute_metrics(
+                    lg, targets, loss_mask, prev_correct, step, ttt_step_loss_decay,
+                    loss_config=loss_config, target_stats_cache=stats_cache, total_in=loss, return_tokens=True)
+                if fuse:
+                    logits = lg.logits
+                metrics.update(s_metrics)
+                draft_tokens.append(tokens)
             else:
                 draft_tokens.append(MT.argmax_rows(logits.detach()))
 
             if self.keep_logits:
                 self.last_logits.append(logits.detach())
-            input_ids = torch.cat(
-                [original_ids[:, 1 + step:], original_ids.new_zeros(1, 1 + step)], dim=-1)
             if full_mask is not None:
                 full_mask = full_mask.extended()
             if sw_mask is not None:
@@ -441,6 +437,8 @@ class Eagle3DraftModel(nn.Module):
 
         if not return_loss:
             return draft_tokens
+        if loss is None:
+            loss = torch.zeros((), device=device)
         metrics["loss_sum"] = loss.detach().clone()
         metrics["loss_total"] = torch.ones((), device=device)
         return draft_tokens, loss, metrics

@@ -44,7 +44,8 @@ class StepPass:
     ``d2t`` (int64 ``[Vd]``): the targets are FULL-vocabulary verifier rows and target element i
     is read at column ``i + d2t[i]`` while streaming; the draft-vocabulary rows come back in
     ``gathered`` (``[rows, Vd]``) for the later steps and the backward.
-    ``counts`` (int32 ``[3]``, zeroed): the acceptance chain is done row by row in the same pass
+    ``counts`` (int32 ``[3]``, zeroed -- or, with ``clear_counts``, cleared by the kernel that maps the rows in
+    front of the one-pass form, the only one that may then run): the acceptance chain is done row by row in the same pass
     (``mask`` / ``prev`` are the step's 1-D views, ``prev`` is updated in place).
     ``grad_in_pass``: a promise of the caller that the reduction behind the row losses gives a row
     whose ``mask`` entry is zero the weight zero (the masked mean of ``compute_metrics`` does).  The
@@ -58,6 +59,7 @@ class StepPass:
     prev: torch.Tensor | None = None
     counts: torch.Tensor | None = None
     grad_in_pass: bool = False
+    clear_counts: bool = False
 
 
 def fused_loss_forward(op: int, logits: torch.Tensor, targets: torch.Tensor, target_stats=None,
@@ -238,8 +240,10 @@ def _loss_forward_with_grad(op, x, y, known, step):
     the front.  Returns ``(loss, lse_t, am_d, am_t, packed, row_map, count)``."""
     rows, vocab = x.shape
     dev = x.device
-    mask_f = step.mask if step.mask.dtype == torch.float32 else step.mask.to(torch.float32)
-    row_map, count = _packed_row_map(mask_f.contiguous())
+    out = torch.empty(rows + 1, device=dev, dtype=torch.int32)
+    row_map, count = out[:rows], out[rows:]
+    _lib.call("spx_mask_row_map", step.mask, _lib.kind_code(step.mask), rows, row_map, count,
+              step.counts if step.clear_counts else None, _lib.stream_ptr(dev))
     packed = torch.empty(rows, vocab, device=dev, dtype=torch.bfloat16)
     stats = torch.empty(4, rows, device=dev, dtype=torch.float32)
     arg = torch.empty(2, rows, device=dev, dtype=torch.int32)
@@ -286,63 +290,139 @@ class _HeadFusedLoss(torch.autograd.Function):
         logits = matmul_nt(x2, weight)
         known = (known_lse_t, known_am_t) if known_lse_t is not None else None
         ctx.op, ctx.total_rows = op, logits.shape[0]
-        xs = logits[:n_rows]
-        ys = None if targets is None else _rows_2d(targets)
-        ctx.one_pass = (known is not None or ys is not None) and _one_pass_ok(op, xs, ys, step)
-        if ctx.one_pass:
-            # the rows are read once: loss, statistics, chain and the (unit-weight) logits gradient
-            loss, lse_t, am_d, am_t, packed, row_map, count = _loss_forward_with_grad(op, xs, ys, known, step)
-            ctx.save_for_backward(packed, row_map, count, weight_t)
-        else:
-            loss, lse_d, lse_t, extra, am_d, am_t, x, y = fused_loss_forward(op, xs, targets, known, step)
-            ctx.save_for_backward(x, None if op == OP_CE else y, lse_d, lse_t, extra, am_t, weight_t)
+        loss, lse_d, lse_t, extra, am_d, am_t, x, y = fused_loss_forward(op, logits[:n_rows], targets, known, step)
+        ctx.save_for_backward(x, None if op == OP_CE else y, lse_d, lse_t, extra, am_t, weight_t)
         ctx.mark_non_differentiable(am_d, am_t, lse_t, logits)
         ctx.set_materialize_grads(False)  # no [T, Vd] zeros for the logits, which carry no gradient
         return loss, am_d, am_t, lse_t, logits
 
     @staticmethod
     def backward(ctx, grad_rows, _gd, _gt, _gl, _glogits):
-        from .gemm import matmul_nt
-
         if grad_rows is None:
             return (None,) * 9
-        if ctx.one_pass:
-            packed, row_map, count, weight_t = ctx.saved_tensors
-            g = grad_rows.reshape(-1).to(torch.float32).contiguous()
-            dx_packed = matmul_nt(packed, weight_t, m_live=count)
-            return (_unpack_rows_scaled(dx_packed, row_map, g, ctx.total_rows), None, None, None, None, None,
-                    None, None, None)
-
-        x, y, lse_d, lse_t, extra, am_t, weight_t = ctx.saved_tensors
-        rows, vocab = x.shape
         g = grad_rows.reshape(-1).to(torch.float32).contiguous()
-        row_map, count = _packed_row_map(g)
-        packed = torch.empty(rows, vocab, device=x.device, dtype=x.dtype)
-        _lib.call(
-            "spx_fused_vocab_loss_bwd_packed", ctx.op, x, x.stride(0), y,
-            y.stride(0) if y is not None else 0, rows, vocab, _lib.dtype_code(x),
-            lse_d, lse_t, extra, am_t, g, None,
-            row_map, packed, packed.stride(0), _lib.stream_ptr(x.device),
-        )
-        dx_packed = matmul_nt(packed, weight_t, m_live=count)
-        return (_unpack_rows(dx_packed, row_map, ctx.total_rows), None, None, None, None, None,
-                None, None, None)
+        return (_head_rows_backward(ctx.op, ctx.saved_tensors, g, ctx.total_rows),) + (None,) * 8
 
 
-def head_fused_rows(op: int, x, weight, weight_t, targets, target_stats=None, n_rows=None, step=None):
-    """``fused_rows`` with the frozen head in front: ``x [1, T, H]`` instead of logits.  Returns
-    ``(row_loss [1, n_rows], argmax_draft, argmax_target, lse_target, logits [1, T, Vd])``."""
+def _head_rows_backward(op, saved, g, total_rows):
+    """dx of the frozen head behind the row losses whose gradients are ``g`` (f32 ``[rows]``)."""
+    from .gemm import matmul_nt
+
+    x, y, lse_d, lse_t, extra, am_t, weight_t = saved
+    rows, vocab = x.shape
+    row_map, count = _packed_row_map(g)
+    packed = torch.empty(rows, vocab, device=x.device, dtype=x.dtype)
+    _lib.call(
+        "spx_fused_vocab_loss_bwd_packed", op, x, x.stride(0), y,
+        y.stride(0) if y is not None else 0, rows, vocab, _lib.dtype_code(x),
+        lse_d, lse_t, extra, am_t, g, None,
+        row_map, packed, packed.stride(0), _lib.stream_ptr(x.device),
+    )
+    dx_packed = matmul_nt(packed, weight_t, m_live=count)
+    return _unpack_rows(dx_packed, row_map, total_rows)
+
+
+@dataclass
+class MeanTerm:
+    """The masked mean behind the row losses of one step (``spx_ttt_step_total``): the step's ``weight``, the
+    term's ``factor`` in the loss, and ``out``, which receives the step's scalars (f32 ``[8]``)."""
+
+    mask: torch.Tensor | None
+    weight: float
+    factor: float
+    out: torch.Tensor
+
+    def reduce(self, loss, am_d, am_t, counts, total_in):
+        """``(total 0-d, row weights)``: ``total_in`` (or nothing) + the weighted masked mean."""
+        n, dev = loss.numel(), loss.device
+        row_weight = torch.empty(n, device=dev, dtype=torch.float32)
+        total = torch.empty((), device=dev, dtype=torch.float32)
+        _lib.call("spx_ttt_step_total", loss, am_d, am_t, self.mask,
+                  _lib.kind_code(self.mask) if self.mask is not None else 0, None, 0, n, self.weight, counts,
+                  self.factor, total_in, total, self.out, row_weight, _lib.stream_ptr(dev))
+        return total, row_weight
+
+
+class _HeadStepLoss(torch.autograd.Function):
+    """``_HeadFusedLoss`` and the masked mean behind it as one node, which also adds the step to the loss so far:
+    ``(x, total_in) -> (total, argmax_draft, argmax_target, lse_target, logits)``.
+
+    Where it can (``_one_pass_ok``) the forward reads the rows once for everything: loss, statistics, acceptance
+    chain and the unit-weight logits gradient of the unmasked rows, packed to the front; the backward is then the
+    input-gradient product of the head and the unpacking of its rows, which applies the row weights."""
+
+    @staticmethod
+    def forward(ctx, x2, total_in, weight, weight_t, targets, op, known, n_rows, step, mean):
+        from .gemm import matmul_nt
+
+        logits = matmul_nt(x2, weight)
+        ctx.op, ctx.total_rows, ctx.factor = op, logits.shape[0], mean.factor
+        xs = logits[:n_rows]
+        ctx.one_pass = (known is not None or targets is not None) and _one_pass_ok(op, xs, targets, step)
+        if ctx.one_pass:
+            step.counts = torch.empty(3, device=x2.device, dtype=torch.int32)
+            step.clear_counts = True
+            loss, lse_t, am_d, am_t, packed, row_map, count = _loss_forward_with_grad(op, xs, targets, known, step)
+            total, row_weight = mean.reduce(loss, am_d, am_t, step.counts, total_in)
+            ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
+        else:
+            step.counts = torch.zeros(3, device=x2.device, dtype=torch.int32)
+            loss, lse_d, lse_t, extra, am_d, am_t, x, y = fused_loss_forward(op, xs, targets, known, step)
+            total, row_weight = mean.reduce(loss, am_d, am_t, step.counts, total_in)
+            ctx.save_for_backward(x, None if op == OP_CE else y, lse_d, lse_t, extra, am_t, weight_t, row_weight)
+        ctx.mark_non_differentiable(am_d, am_t, lse_t, logits)
+        ctx.set_materialize_grads(False)
+        return total, am_d, am_t, lse_t, logits
+
+    @staticmethod
+    def backward(ctx, g, _gd, _gt, _gl, _glogits):
+        from .gemm import matmul_nt
+
+        if g is None:
+            return (None,) * 10
+        g32 = g.to(torch.float32)
+        if ctx.one_pass:
+            packed, row_map, count, weight_t, row_weight = ctx.saved_tensors
+            dx_packed = matmul_nt(packed, weight_t, m_live=count)
+            dx = torch.empty(ctx.total_rows, dx_packed.shape[1], device=packed.device, dtype=packed.dtype)
+            _lib.call("spx_unpack_rows_graded", dx_packed, dx_packed.stride(0), row_map, row_weight, g32, ctx.factor,
+                      row_map.numel(), ctx.total_rows, dx.shape[1], dx, dx.stride(0), _lib.stream_ptr(dx.device))
+        else:
+            *saved, row_weight = ctx.saved_tensors
+            dx = _head_rows_backward(ctx.op, saved, row_weight * (g32 * ctx.factor), ctx.total_rows)
+        return (dx, g if ctx.needs_input_grad[1] else None) + (None,) * 8
+
+
+def head_step_loss(op: int, x, weight, weight_t, targets, target_stats, n_rows: int, step: StepPass, mean: MeanTerm,
+                   total_in=None):
+    """``head_fused_rows`` of one step with its masked mean (``mean``) added to ``total_in``: ``(total, argmax_draft,
+    argmax_target, lse_target, logits [1, T, Vd])``, the row quantities ``[n_rows]``."""
+    y = _check_head(x, weight, targets, n_rows)
+    t = x.shape[1]
+    total, am_d, am_t, lse_t, logits = _HeadStepLoss.apply(x.reshape(t, x.shape[2]), total_in, weight, weight_t, y, op,
+                                                           target_stats, n_rows, step, mean)
+    return total, am_d, am_t, lse_t, logits.view(1, t, weight.shape[0])
+
+
+def _check_head(x, weight, targets, n: int):
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise _lib.SpxError("head_fused_rows takes bf16 operands")
     if weight.requires_grad:
         raise ValueError("head_fused_rows is for a frozen head (no weight gradient is produced)")
     if x.dim() != 3 or x.shape[0] != 1:
         raise ValueError("x must be [1, T, H] (the packed batch layout)")
-    t = x.shape[1]
-    n = t if n_rows is None else int(n_rows)
     y = None if targets is None else _rows_2d(targets)
     if y is not None and y.shape[0] != n:
         raise ValueError(f"targets have {y.shape[0]} rows, expected {n}")
+    return y
+
+
+def head_fused_rows(op: int, x, weight, weight_t, targets, target_stats=None, n_rows=None, step=None):
+    """``fused_rows`` with the frozen head in front: ``x [1, T, H]`` instead of logits.  Returns
+    ``(row_loss [1, n_rows], argmax_draft, argmax_target, lse_target, logits [1, T, Vd])``."""
+    n = x.shape[1] if n_rows is None else int(n_rows)
+    y = _check_head(x, weight, targets, n)
+    t = x.shape[1]
     ks = (None, None) if target_stats is None else (target_stats[0], target_stats[1])
     # (a view, not x[0]: the backward of a select writes the gradient into a zero-filled copy)
     loss, am_d, am_t, lse_t, logits = _HeadFusedLoss.apply(x.reshape(t, x.shape[2]), weight, weight_t, y, op,

@@ -25,38 +25,23 @@ def _as_mask(t: torch.Tensor) -> torch.Tensor:
 
 
 class _StepReduce(torch.autograd.Function):
-    """(row_loss [n] f32) -> weighted masked mean (0-d); also fills ``out`` (6 floats)
-    and updates ``prev_correct`` in place.  d/d row_loss = row_weight.  With ``counts`` (int32
-    ``[3]``) the acceptance chain was already done by the loss pass (``losses.StepPass``): only
-    the mean is reduced here and the counts are copied into ``out``."""
+    """(row_loss [n] f32, total_in) -> total_in + factor * weighted masked mean (0-d); also fills the mean's
+    ``out`` and, where the loss pass has not done the acceptance chain (no ``counts``), leaves it out:
+    d/d row_loss = factor * row_weight."""
 
     @staticmethod
-    def forward(ctx, row_loss, am_d, am_t, mask, prev, weight, out, counts=None):
-        n = row_loss.numel()
-        row_loss = row_loss.reshape(-1).contiguous()
-        row_weight = torch.empty(n, device=row_loss.device, dtype=torch.float32)
-        if counts is not None:
-            _lib.call(
-                "spx_ttt_step_mean", row_loss, mask,
-                _lib.kind_code(mask) if mask is not None else 0, n, float(weight), counts,
-                out, row_weight, _lib.stream_ptr(row_loss.device),
-            )
-        else:
-            _lib.call(
-                "spx_ttt_step_reduce", row_loss, am_d, am_t,
-                mask, _lib.kind_code(mask) if mask is not None else 0,
-                prev, _lib.kind_code(prev) if prev is not None else 0,
-                n, float(weight), out, row_weight,
-                _lib.stream_ptr(row_loss.device),
-            )
+    def forward(ctx, row_loss, total_in, am_d, am_t, mean, counts):
+        shape = row_loss.shape
+        total, row_weight = mean.reduce(row_loss.reshape(-1).contiguous(), am_d, am_t, counts, total_in)
         ctx.save_for_backward(row_weight)
-        ctx.shape = row_loss.shape
-        return out[0].clone()
+        ctx.shape, ctx.factor = shape, mean.factor
+        return total
 
     @staticmethod
     def backward(ctx, g):
         (row_weight,) = ctx.saved_tensors
-        return (row_weight * g).view(ctx.shape), None, None, None, None, None, None, None
+        scaled = g if ctx.factor == 1.0 else g * ctx.factor
+        return (row_weight * scaled).view(ctx.shape), g if ctx.needs_input_grad[1] else None, None, None, None, None
 
 
 class TargetGather:
@@ -141,17 +126,19 @@ class Head:
 
 def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
                     ttt_step_loss_decay: float, loss_config: L.LossConfig | None = None,
-                    target_stats_cache: dict | None = None, return_pred: bool = False):
+                    target_stats_cache: dict | None = None, return_pred: bool = False,
+                    total_in: torch.Tensor | None = None, return_tokens: bool = False):
     """EAGLE3 per-step loss + metrics; same contract as models/eagle3/metrics.py:51-119.
 
     ``prev_correct`` (any mask dtype) is updated in place.  Returns
     ``(loss 0-d, metrics dict of 0-d tensors)``.
 
-    Two optional extras beyond the reference contract: ``target_stats_cache`` (a dict the
+    Optional extras beyond the reference contract: ``target_stats_cache`` (a dict the
     caller keeps across the TTT steps of ONE forward) lets steps >= 1 reuse the verifier
     rows' log-sum-exp / arg-max computed at step 0 (``targets`` is the same tensor at every
     step, only shifted); ``return_pred=True`` also returns the draft arg-max of the aligned
-    rows (int32 ``[T - ttt_step]``).
+    rows (int32 ``[T - ttt_step]``), ``return_tokens=True`` that of all rows (int64 ``[1, T]``: the last ``ttt_step``
+    rows have no target); ``total_in`` (0-d) is added to the returned loss, not to its metric.
     """
     if loss_config is None:
         loss_config = {"kl_div": (L.kl_div_loss, 1.0)}
@@ -164,7 +151,7 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
                   and logits.weight_t is not None)
         if single:
             head = logits
-            logits = torch.empty(1, head.x.shape[1], 0, device=head.x.device)  # shape carrier only
+            logits = head.x[:, :, :0].detach()  # shape carrier only
         else:
             logits = logits.materialize()
     if logits.shape[0] != 1:
@@ -201,19 +188,22 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
         if prev1.stride(0) != 1:
             raise ValueError("prev_correct must be contiguous (it is updated in place)")
 
-    total = None
-    terms = {}
     multi = len(loss_config) > 1
+    # (one term: its mean goes straight onto the loss so far; several: onto each other first)
+    total = None if multi else total_in
+    terms = {}
     first_out = None
     counts = None
     for ti, (name, (fn, w)) in enumerate(loss_config.items()):
-        out = torch.empty(6, device=dev, dtype=torch.float32)
+        out = torch.empty(8, device=dev, dtype=torch.float32)
+        mean = L.MeanTerm(mask1, weight, float(w), out)
         op = L.PRIMITIVE_OP.get(name)
         step = None
         if ti == 0:
             # the first term's row pass also gathers the targets (first step of a TargetGather)
             # and advances the acceptance chain
-            counts = torch.zeros(3, device=dev, dtype=torch.int32)
+            if head is None:
+                counts = torch.zeros(3, device=dev, dtype=torch.int32)
             # (a row the mask removes has weight zero in the masked mean below: the head + loss node may
             # write the logits gradient of the other rows in the same pass)
             step = L.StepPass(d2t=gather.d2t if gather is not None else None, mask=mask1, prev=prev1,
@@ -230,9 +220,8 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
                     known = (full[0][ttt_step:], full[1][ttt_step:])
             # the full logits go in with a row count: see _FusedLoss.forward
             if head is not None:
-                rows, am_d, am_t, lse_t, head.logits = L.head_fused_rows(
-                    op, head.x, head.weight, head.weight_t, s_targets, known, n_rows=s_logits.shape[1],
-                    step=step)
+                total, am_d, am_t, lse_t, head.logits = L.head_step_loss(
+                    op, head.x, head.weight, head.weight_t, s_targets, known, s_logits.shape[1], step, mean, total)
             else:
                 rows, am_d, am_t, lse_t = L.fused_rows(op, logits, s_targets, known,
                                                        n_rows=s_logits.shape[1], step=step)
@@ -248,16 +237,21 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
         if ti == 0:
             pred = am_d.reshape(-1)
         # only the first term advances the acceptance chain (inside its row pass)
-        term = _StepReduce.apply(rows.reshape(-1), am_d.reshape(-1), am_t.reshape(-1), mask1,
-                                 None, weight, out, counts if ti == 0 else None)
+        if head is None:
+            total = _StepReduce.apply(rows.reshape(-1), total, am_d.reshape(-1), am_t.reshape(-1), mean,
+                                      counts if ti == 0 else None)
         if ti == 0:
             first_out = out
         if multi:
-            terms[f"{name}_loss"] = term.detach()
-        total = w * term if total is None else total + w * term
+            terms[f"{name}_loss"] = out[0]
 
-    one = torch.ones((), device=dev)
-    m = {f"loss_{ttt_step}_sum": total.detach().clone(), f"loss_{ttt_step}_total": one}
+    one = first_out[7]
+    if multi:
+        m = {f"loss_{ttt_step}_sum": total.detach().clone(), f"loss_{ttt_step}_total": one}
+        if total_in is not None:
+            total = total_in + total
+    else:
+        m = {f"loss_{ttt_step}_sum": first_out[6], f"loss_{ttt_step}_total": one}
     for tname, tval in terms.items():
         m[f"{tname}_{ttt_step}_sum"] = tval
         m[f"{tname}_{ttt_step}_total"] = one.clone()
@@ -265,27 +259,27 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
     m[f"full_acc_{ttt_step}_total"] = first_out[2]
     m[f"cond_acc_{ttt_step}_sum"] = first_out[3]
     m[f"cond_acc_{ttt_step}_total"] = first_out[4]
+    if return_tokens:
+        return total, m, row_tokens(pred, (logits if head is None else head.logits).detach()[0, s_logits.shape[1]:])
     if return_pred:
         return total, m, pred
     return total, m
 
 
+def row_tokens(known, rows: torch.Tensor) -> torch.Tensor:
+    """int64 ``[1, n + tail]``: the arg-maxes ``known`` (int32 ``[n]`` or None) and those of ``rows [tail, V]``."""
+    n = 0 if known is None else known.numel()
+    rows = L._rows_2d(rows)
+    tail, vocab = rows.shape
+    out = torch.empty(1, n + tail, device=rows.device, dtype=torch.int64)
+    _lib.call("spx_row_tokens", known, n, rows if tail else None, rows.stride(0), tail, vocab, _lib.dtype_code(rows),
+              out, _lib.stream_ptr(rows.device))
+    return out
+
+
 def argmax_rows(logits: torch.Tensor) -> torch.Tensor:
-    """First-index arg-max over the last axis as int64, through the loss kernel's
-    arg-max path (pairs every row with itself)."""
-    x = L._rows_2d(logits)
-    rows, vocab = x.shape
-    dev = x.device
-    scratch = torch.empty(4, max(rows, 1), device=dev, dtype=torch.float32)
-    out = torch.empty(max(rows, 1), device=dev, dtype=torch.int32)
-    if rows:
-        _lib.call(
-            "spx_fused_vocab_loss_fwd", L.OP_CE, x, x.stride(0), x,
-            x.stride(0), rows, vocab, _lib.dtype_code(x), scratch[0],
-            scratch[1], scratch[2], scratch[3], out,
-            None, 0, _lib.stream_ptr(dev),
-        )
-    return out[:rows].to(torch.int64).view(logits.shape[:-1])
+    """First-index arg-max over the last axis as int64."""
+    return row_tokens(None, L._rows_2d(logits)).view(logits.shape[:-1])
 
 
 class _BlockReduce(torch.autograd.Function):

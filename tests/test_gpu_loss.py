@@ -529,3 +529,43 @@ def test_pipelined_gather_pass_on_the_edges_of_its_tiling(op_name, case):
         assert torch.equal(a, b), name
     assert torch.equal(prev_got, prev_ref)
     assert step.counts.tolist() == [int(out[1]), int(out[2]), int(out[4])]
+
+
+@pytest.mark.parametrize("n,tail,vocab,dtype", [(0, 3, 5, torch.float32), (1, 0, 8, torch.bfloat16),
+                                                (255, 1, 2047, torch.bfloat16), (257, 4, 32000, torch.bfloat16),
+                                                (300, 2, 2056, torch.float32)])
+def test_row_tokens_widen_the_known_and_find_the_rest(n, tail, vocab, dtype):
+    from speculators_amd.metrics import row_tokens
+
+    g = torch.Generator().manual_seed(n + vocab)
+    known = torch.randint(0, vocab, (n,), generator=g, dtype=torch.int32)
+    rows = torch.randint(-4, 5, (n + tail, vocab), generator=g).to(dtype)  # many equal maxima: the first one counts
+    got = row_tokens(known.cuda(), rows.cuda()[n:])
+    want = torch.cat([known.long(), torch.tensor([int((r == r.max()).nonzero()[0]) for r in rows[n:].float()],
+                                                 dtype=torch.int64)])
+    assert got.shape == (1, n + tail) and torch.equal(got[0].cpu(), want)
+
+
+@pytest.mark.parametrize("rows", [1, 1023, 1025, 3000])
+@pytest.mark.parametrize("kind", [torch.bool, torch.int64, torch.bfloat16])
+def test_mask_row_map_and_step_total(rows, kind):
+    from speculators_amd import _lib
+
+    g = torch.Generator().manual_seed(rows)
+    mask = (torch.rand(rows, generator=g) < 0.6).to(kind).cuda()
+    out = torch.full((rows + 4,), 7, device="cuda", dtype=torch.int32)
+    st = _lib.stream_ptr(mask.device)
+    _lib.call("spx_mask_row_map", mask, _lib.kind_code(mask), rows, out, out[rows:], out[rows + 1:], st)
+    live = mask.cpu().float() != 0
+    want = torch.where(live, live.long().cumsum(0) - 1, torch.tensor(-1))
+    assert torch.equal(out[:rows].cpu().long(), want) and out[rows:].tolist() == [int(live.sum()), 0, 0, 0]
+    loss = torch.randn(rows, generator=g).cuda()
+    counts = torch.tensor([3, 5, 9], device="cuda", dtype=torch.int32)
+    a, b = torch.empty(8, device="cuda"), torch.empty(6, device="cuda")
+    rw = torch.empty(2, rows, device="cuda")
+    before, total = torch.tensor(2.5, device="cuda"), torch.empty((), device="cuda")
+    _lib.call("spx_ttt_step_mean", loss, mask, _lib.kind_code(mask), rows, 0.7, counts, b, rw[0], st)
+    _lib.call("spx_ttt_step_total", loss, None, None, mask, _lib.kind_code(mask), None, 0, rows, 0.7, counts, 0.25,
+              before, total, a, rw[1], st)
+    assert torch.equal(a[:6], b) and torch.equal(rw[0], rw[1]) and a[7].item() == 1.0
+    assert a[6].item() == b[0].item() * 0.25 and abs(total.item() - (2.5 + a[6].item())) < 1e-6
