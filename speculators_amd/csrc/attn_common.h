@@ -8,7 +8,7 @@
 // cross-half shuffle, and the probabilities feed the second product
 // O^T = V^T P^T directly as the B operand (a lane's registers 8s..8s+7 are the
 // eight k-slots of the 16-key step s).  The A operand of that product needs V
-// with keys contiguous, so V is transposed once per call into a workspace.
+// with keys contiguous: it comes out of the row-major V tile through transposing LDS reads.
 #pragma once
 
 #include "spx_common.h"
@@ -18,8 +18,6 @@ namespace spx {
 constexpr int kAttnThreads = 256;
 constexpr int kBM = 128;  // query rows per workgroup
 constexpr int kBN = 64;   // keys per tile
-constexpr int kKPad = 8;  // K tile row stride = D + 8 elements  (272 B at D=128)
-constexpr int kVPad = 8;  // V^T tile row stride = 64 + 8 elements (144 B: 16-byte aligned rows)
 
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);

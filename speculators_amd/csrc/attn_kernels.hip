@@ -16,6 +16,7 @@
 // Key tiles that no row of a workgroup can see are skipped analytically; no
 // dense mask or BlockMask exists anywhere.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -35,21 +36,34 @@ struct AttnParams {
 };
 
 // ---------------------------------------------------------------- mask descriptors
+// largest value of the lower threads of a workgroup of 1024 (-1: none)
+__device__ __forceinline__ int lower_max(int v) {
+  __shared__ int wave_top[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(v, d, 64);
+    if (lane >= d) v = max(v, o);
+  }
+  if (lane == 63) wave_top[wave] = v;
+  __syncthreads();
+  const int up = __shfl_up(v, 1, 64);
+  int carry = lane > 0 ? up : -1;
+  for (int w = 0; w < wave; ++w) carry = max(carry, wave_top[w]);
+  return carry;
+}
+
+// (one workgroup: a walk over the run starts of up to 1023 lower threads in LDS made this 8.5 us at any length)
 template <typename I>
 __global__ __launch_bounds__(1024) void ttt_row_lo_kernel(const I* __restrict__ doc, int64_t T,
                                                           int64_t window, int32_t* __restrict__ lo) {
-  __shared__ int seg_max[1024];
   const int t = threadIdx.x;
   const int64_t len = (T + 1023) / 1024;
   const int64_t b = t * len, e = (b + len < T) ? b + len : T;
   int run = -1;
   for (int64_t i = b; i < e; ++i)
     if (i == 0 || doc[i] != doc[i - 1]) run = (int)i;
-  seg_max[t] = run;
-  __syncthreads();
-  int carry = -1;
-  for (int s = 0; s < t; ++s) carry = max(carry, seg_max[s]);
-  run = carry;
+  run = lower_max(run);
   for (int64_t i = b; i < e; ++i) {
     if (i == 0 || doc[i] != doc[i - 1]) run = (int)i;
     int v = run;
@@ -63,18 +77,13 @@ __global__ __launch_bounds__(1024) void ttt_row_lo_kernel(const I* __restrict__ 
 template <typename I>
 __global__ __launch_bounds__(1024) void doc_run_start_kernel(const I* __restrict__ doc, int64_t T,
                                                              int32_t* __restrict__ start) {
-  __shared__ int seg_max[1024];
   const int t = threadIdx.x;
   const int64_t len = (T + 1023) / 1024;
   const int64_t b = t * len, e = (b + len < T) ? b + len : T;
   int run = -1;
   for (int64_t i = b; i < e; ++i)
     if (i == 0 || doc[i] != doc[i - 1]) run = (int)i;
-  seg_max[t] = run;
-  __syncthreads();
-  int carry = -1;
-  for (int s = 0; s < t; ++s) carry = max(carry, seg_max[s]);
-  run = carry;
+  run = lower_max(run);
   for (int64_t i = b; i < e; ++i) {
     if (i == 0 || doc[i] != doc[i - 1]) run = (int)i;
     start[i] = run;
@@ -129,13 +138,9 @@ __device__ __forceinline__ u32x4 scale_bf16x8(u32x4 raw, float c) {
 // (eight lanes read a whole 128-byte line), transposes it in registers (v_perm_b32) and writes, for each
 // of its 8 columns, the two 4-row halves of the block to their permuted places (8 bytes each; the eight
 // lanes that share a column fill its 128-byte line in two store instructions).  cols a multiple of 8.
-// SCALED: the elements are multiplied by `scale` first (scale_bf16x8) and the scaled rows are also
-// written row-major to `scaled` ([h][rows][cols], head stride rows * cols).
-template <bool SCALED>
 __global__ __launch_bounds__(64) void transpose_bf16_kernel(
     const uint16_t* __restrict__ src, int64_t src_hs, int64_t src_ld, int rows, int cols,
-    uint16_t* __restrict__ dst, int64_t dst_hs, int64_t ld_dst, float scale,
-    uint16_t* __restrict__ scaled) {
+    uint16_t* __restrict__ dst, int64_t dst_hs, int64_t ld_dst) {
   const int h = blockIdx.z;
   const int lane = threadIdx.x;
   const int rb = lane >> 3, cb = lane & 7;
@@ -147,13 +152,7 @@ __global__ __launch_bounds__(64) void transpose_bf16_kernel(
   for (int j = 0; j < 8; ++j) {
     const u32x4 z = {0, 0, 0, 0};
     in[j] = (r0 + j < rows) ? *reinterpret_cast<const u32x4*>(s + (int64_t)(r0 + j) * src_ld) : z;
-    if (SCALED) {
-      in[j] = scale_bf16x8(in[j], scale);
-      if (r0 + j < rows)
-        *reinterpret_cast<u32x4*>(scaled + ((int64_t)h * rows + r0 + j) * cols + c0) = in[j];
-    }
   }
-  if (SCALED && dst == nullptr) return;  // only the scaled row-major copy is wanted
   // where the block's two halves go: r0 % 16 == 0 -> r0 and r0 + 8, r0 % 16 == 8 -> r0 - 4 and r0 + 4
   const int p_lo = (r0 & 8) ? r0 - 4 : r0, p_hi = (r0 & 8) ? r0 + 4 : r0 + 8;
   uint16_t* d = dst + (int64_t)h * dst_hs + (int64_t)c0 * ld_dst;
@@ -248,6 +247,17 @@ __device__ __forceinline__ void load_bounds(const AttnParams& p, const int (&ic)
   rb.blk_a2 = uni(rb.blk_a2); rb.blk_b2 = uni(rb.blk_b2);
 }
 
+// Four 16-bit values per lane from LDS, transposed inside every group of 16 lanes: lane 4u + w of
+// a group receives, as element j, element w of the 8 bytes that lane 4j + u of the group points at.
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef short i16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ i16x4 lds_tr16(uint32_t addr) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(uintptr_t)addr);
+}
+__device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
+  return lds_tr16((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)p);
+}
+
 // Passes a score block through an empty volatile asm statement.  Placed inside the branch that
 // masks a tile it keeps the compiler from turning that branch into selects which every tile, masked
 // or not, would then execute (96 vector instructions per tile): volatile asm is never speculated.
@@ -281,44 +291,36 @@ struct PrioPair {
 #define SPX_DQ_PRIO_VALU() PrioPair<prio_first(SPX_DQ_PRIO), prio_second(SPX_DQ_PRIO)>::vector()
 #define SPX_DKV_PRIO_MFMA() PrioPair<prio_first(SPX_DKV_PRIO), prio_second(SPX_DKV_PRIO)>::matrix()
 #define SPX_DKV_PRIO_VALU() PrioPair<prio_first(SPX_DKV_PRIO), prio_second(SPX_DKV_PRIO)>::vector()
-#define SPX_DKV_REMAT 1
 #define SPX_FWD_MINB 2
 #define SPX_DQ_MINB 2
-#define SPX_DKV_MINB 1
-// How the forward kernel brings a key tile into LDS: through registers at the point of use (0),
-// through registers one tile ahead (1), or with global -> LDS loads into the other of two tile
-// buffers (2).  A 16-byte LDS write from registers holds the LDS pipe twice as long as a 16-byte
-// read, and these kernels keep that pipe busy all the time: mode 2 takes the writes off it.
-template <int D, int NW, int PF>
+// A key tile is 64 rows of K and of V as they lie in memory, brought global -> LDS directly into the other of two tile
+// buffers: a 16-byte LDS write from registers holds the LDS pipe twice as long as a 16-byte read, and these kernels keep
+// that pipe busy all the time.  The transposed operand of the second product comes out of the row-major tile through
+// transposing LDS reads (dQ: K^T; forward, TR: V^T), or, in larger forward calls, out of a copy V^T made once per call: two
+// 8-byte reads for one of 16 cost the forward 6 % at head_dim 128 and 20 % at 256, the copy is a launch of 4 us (fwd_tr).
+template <int D, int NW>
 struct FwdSmem {
-  static constexpr int KS = D + kKPad, VS = kBN + kVPad;
-  static constexpr int kTileK = kBN * D * 2, kTileV = D * kBN * 2;  // mode 2: unpadded, swizzled
-  static constexpr int kBuf = kTileK + kTileV;
-  static constexpr int kTiles = PF == 2 ? 2 * kBuf : (kBN * KS + D * VS) * 2;
+  static constexpr int kTile = kBN * D * 2;  // unpadded, swizzled
+  static constexpr int kBuf = 2 * kTile;     // K, V
+  static constexpr int kTiles = 2 * kBuf;
   static constexpr int kBytes = kTiles + 4 * NW * (int)sizeof(int);
 };
 
 // operand fragments in flight per product (registers: 4 per fragment): the LDS pipe delivers
 // well over 150 B/clk per CU, what a wave waits for is the latency of its own reads
 #define SPX_FWD_RING 8
-template <int D, int NSB, int NW, int PF>
+template <int D, int NSB, int NW, bool TR>
 __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_kernel(AttnParams p,
                                                                 const uint16_t* __restrict__ Vt,
                                                                 uint16_t* __restrict__ O,
                                                                 float* __restrict__ LSE) {
-  using SM = FwdSmem<D, NW, PF>;
-  constexpr int KS = SM::KS;
-  constexpr int VS = SM::VS;
+  using SM = FwdSmem<D, NW>;
   constexpr int NKK = D / 16;
   constexpr int NDB = D / 32;
-  constexpr int NT = 64 * NW;
-  constexpr int CPT = (kBN * D / 8) / NT;
   constexpr int BMW = 32 * NSB;
   constexpr int BM = NW * BMW;
 
   extern __shared__ __attribute__((aligned(16))) uint8_t fwd_smem[];
-  uint16_t* const Ks = reinterpret_cast<uint16_t*>(fwd_smem);
-  uint16_t* const Vs = Ks + kBN * KS;
   int* const red = reinterpret_cast<int*>(fwd_smem + SM::kTiles);
 
   const int group = p.Hq / p.Hkv;
@@ -377,60 +379,25 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
   }
 
   const uint16_t* Kh = p.K + (int64_t)kvh * p.k_hs;
-  const uint16_t* Vth = Vt + (int64_t)kvh * D * p.NKVp;
+  const uint16_t* Vh = p.V + (int64_t)kvh * p.v_hs;
   const int last_row = p.NKV - 1;
 
-  u32x4 kreg[CPT], vreg[CPT];
-  auto fetch = [&](int n0) {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      const int kr = min(n0 + krow, last_row);
-      kreg[n] = *reinterpret_cast<const u32x4*>(Kh + (int64_t)kr * D + kcol);
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      vreg[n] = *reinterpret_cast<const u32x4*>(Vth + (int64_t)vd * p.NKVp + n0 + vcol);
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      *reinterpret_cast<u32x4*>(&Ks[krow * KS + kcol]) = kreg[n];
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      *reinterpret_cast<u32x4*>(&Vs[vd * VS + vcol]) = vreg[n];
-    }
-  };
-
-  auto direct = [&](int n0) {  // global -> LDS without holding the tile in registers
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      const int kr = min(n0 + krow, last_row);
-      *reinterpret_cast<u32x4*>(&Ks[krow * KS + kcol]) =
-          *reinterpret_cast<const u32x4*>(Kh + (int64_t)kr * D + kcol);
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      const u32x4 t = *reinterpret_cast<const u32x4*>(Vth + (int64_t)vd * p.NKVp + n0 + vcol);
-      *reinterpret_cast<u32x4*>(&Vs[vd * VS + vcol]) = t;
-    }
-  };
-
-  // ---- mode 2: tiles as 1 KB wave loads global -> LDS.  K tile: rows of D * 2 bytes, V^T tile: rows
-  // of 128 bytes; the 16-byte chunk c of row r lives in slot c ^ swz(r), which makes the fragment
-  // reads (32 lanes = 32 rows, one logical chunk) conflict free without padding.
-  constexpr int RBK = D * 2, CKK = RBK / 16;             // bytes and chunks per K row
-  constexpr int LPK = (kBN * RBK / 1024) / NW;           // wave loads per wave: K tile
-  constexpr int LPV = (D * 128 / 1024) / NW;             // V^T tile
+  // ---- tiles as 1 KB wave loads global -> LDS: rows of D * 2 bytes (V^T: 128 bytes), the 16-byte chunk c of row r in
+  // slot c ^ swz(r).  K and V^T (32 lanes = 32 rows, one chunk) and V (transposing reads: 4 + 4 rows x 64 bytes, see the dQ
+  // kernel) are read differently and swizzled for their own kind of read: conflict free without padding.
+  constexpr int RBK = D * 2, CKK = RBK / 16;             // bytes and chunks per row
+  constexpr int LPK = (kBN * RBK / 1024) / NW;           // wave loads per wave and tile
   auto swz_k = [](int r) { return CKK == 8 ? (r >> 1) & 7 : r & 15; };
-  auto swz_v = [](int r) { return (r >> 1) & 7; };
+  auto swz_v = [](int r) { return CKK == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3); };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)fwd_smem;
-  u32x4 kres, vres;
-  int k_row[PF == 2 ? LPK : 1], k_col[PF == 2 ? LPK : 1], v_off[PF == 2 ? LPV : 1];
-  if constexpr (PF == 2) {
-    kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
-    vres = make_rsrc(Vth, (uint32_t)((int64_t)D * p.NKVp * 2));
+  const u32x4 kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
+  const uint16_t* const Vth = Vt + (int64_t)kvh * D * p.NKVp;
+  const u32x4 vres = TR ? make_rsrc(Vh, (uint32_t)((int64_t)p.NKV * RBK))
+                        : make_rsrc(Vth, (uint32_t)((int64_t)D * p.NKVp * 2));
+  constexpr int LPV = (D * 128 / 1024) / NW;             // V^T tile
+  auto swz_vt = [](int r) { return (r >> 1) & 7; };
+  int k_row[TR ? 1 : LPK], k_col[TR ? 1 : LPK], v_off[TR ? 1 : LPV];
+  if constexpr (!TR) {
 #pragma unroll
     for (int j = 0; j < LPK; ++j) {
       const int r = (wave * LPK + j) * (1024 / RBK) + lane / CKK;
@@ -440,11 +407,11 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
 #pragma unroll
     for (int j = 0; j < LPV; ++j) {
       const int r = (wave * LPV + j) * 8 + lane / 8;
-      v_off[j] = r * p.NKVp * 2 + ((lane & 7) ^ swz_v(r)) * 16;
+      v_off[j] = r * p.NKVp * 2 + ((lane & 7) ^ swz_vt(r)) * 16;
     }
   }
   auto issue = [&](int n0, int buf) __attribute__((always_inline)) {
-    if constexpr (PF == 2) {
+    if constexpr (!TR) {
       const uint32_t kb = lds0 + buf * SM::kBuf + wave * LPK * 1024;
       if (n0 + kBN <= p.NKV) {
         // every row of the tile exists: the lane's offset inside a tile is loop invariant, the tile's
@@ -452,37 +419,71 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
 #pragma unroll
         for (int j = 0; j < LPK; ++j) load_to_lds16<0>(kres, kb + j * 1024, k_row[j] * RBK + k_col[j], n0 * RBK);
       } else {
-        // the last, ragged tile: rows past the end repeat the last one (they are masked out)
 #pragma unroll
         for (int j = 0; j < LPK; ++j)
           load_to_lds16<0>(kres, kb + j * 1024, min(n0 + k_row[j], last_row) * RBK + k_col[j], 0);
       }
-      const uint32_t vb = lds0 + buf * SM::kBuf + SM::kTileK + wave * LPV * 1024;
+      const uint32_t vb = lds0 + buf * SM::kBuf + SM::kTile + wave * LPV * 1024;
 #pragma unroll
       for (int j = 0; j < LPV; ++j) load_to_lds16<0>(vres, vb + j * 1024, v_off[j], n0 * 2);
+      return;
+    }
+    // (offsets recomputed per tile: four vector instructions per load against 2 LPK registers)
+    int lane_v = lane;
+    if (D > 64) asm volatile("" : "+v"(lane_v));
+    const uint32_t kb = lds0 + buf * SM::kBuf + wave * LPK * 1024, vb = kb + SM::kTile;
+    const bool whole = n0 + kBN <= p.NKV;
+#pragma unroll
+    for (int j = 0; j < LPK; ++j) {
+      const int r = (wave * LPK + j) * (1024 / RBK) + lane_v / CKK;
+      const int ck = ((lane_v % CKK) ^ swz_k(r)) * 16, cv = ((lane_v % CKK) ^ swz_v(r)) * 16;
+      if (whole) {
+        // every row of the tile exists: its first row goes into the scalar offset
+        load_to_lds16<0>(kres, kb + j * 1024, r * RBK + ck, n0 * RBK);
+        load_to_lds16<0>(vres, vb + j * 1024, r * RBK + cv, n0 * RBK);
+      } else {
+        // the last, ragged tile: rows past the end repeat the last one (they are masked out)
+        const int rr = min(n0 + r, last_row) * RBK;
+        load_to_lds16<0>(kres, kb + j * 1024, rr + ck, 0);
+        load_to_lds16<0>(vres, vb + j * 1024, rr + cv, 0);
+      }
     }
   };
-  // fragment reads of mode 2: byte offsets of this lane's row and chunk (step 0) inside a tile
+  // fragment reads: byte offsets of this lane's row and chunk (step 0) inside a K tile
   const int rdk = col * RBK + ((g ^ swz_k(col)) * 16);
-  const int rdv = col * 128 + ((g ^ swz_v(col)) * 16);
+  // ... and of the rows 4 (G >> 1) + (s >> 2) (+ 8) of a 16-key step inside a V tile (lane s of 16-lane group G)
+  const int tG = lane >> 4, ts = lane & 15;
+  const int trow = 4 * (tG >> 1) + (ts >> 2);
+  const int tcl = 2 * (tG & 1) + ((ts & 3) >> 1);
+  const int rt0 = trow * RBK + ((tcl ^ swz_v(trow)) * 16) + (ts & 1) * 8;
+  const int rt1 = (trow + 8) * RBK + ((tcl ^ swz_v(trow + 8)) * 16) + (ts & 1) * 8;
   // The fragment reads as LDS addresses, one register per swizzle term, kept opaque to the
-  // compiler: what is added to them per read (buffer, key half, D block) is a constant and goes
+  // compiler: what is added to them per read (buffer, key half, 16-key step) is a constant and goes
   // into the offset field.  Formed on the symbol of the dynamic array instead, every read costs a
   // vector add of that link-time constant.
   // Only where both tile buffers lie inside the 64 KB an offset field reaches (head_dim <= 128); past
   // that the constants need an add again and the registers are better left to the accumulators.
-  constexpr bool kAbsRd = PF == 2 && 2 * SM::kBuf <= 65536;
-  uint32_t krd[kAbsRd ? NKK : 1], vrd[kAbsRd ? 4 : 1];
+  constexpr bool kAbsRd = 2 * SM::kBuf <= 65536;
+  const int rdv = col * 128 + ((g ^ swz_vt(col)) * 16);
+  uint32_t krd[kAbsRd ? NKK : 1], vrd0[kAbsRd && TR ? NDB : 1], vrd1[kAbsRd && TR ? NDB : 1], vrd[kAbsRd && !TR ? 4 : 1];
   if constexpr (kAbsRd) {
 #pragma unroll
     for (int j = 0; j < NKK; ++j) {
       krd[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
       asm volatile("" : "+v"(krd[j]));
     }
+    if constexpr (!TR) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      vrd[j] = lds0 + (uint32_t)(SM::kTileK + (rdv ^ (j * 32)));
-      asm volatile("" : "+v"(vrd[j]));
+      for (int j = 0; j < 4; ++j) {
+        vrd[j] = lds0 + (uint32_t)(SM::kTile + (rdv ^ (j * 32)));
+        asm volatile("" : "+v"(vrd[j]));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < (TR ? NDB : 0); ++j) {
+      vrd0[j] = lds0 + (uint32_t)(SM::kTile + (rt0 ^ (j * 64)));
+      vrd1[j] = lds0 + (uint32_t)(SM::kTile + (rt1 ^ (j * 64)));
+      asm volatile("" : "+v"(vrd0[j]), "+v"(vrd1[j]));
     }
   }
 
@@ -493,27 +494,17 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
                       int w_bmin, int w_bmax, int blk_a, int blk_b) {
     if (blk_b <= blk_a) return;
     const int n_begin = (blk_a / kBN) * kBN;
-    if (PF == 1) fetch(n_begin);
-    if constexpr (PF == 2) {
-      __syncthreads();  // a previous pass may still be reading either buffer
-      issue(n_begin, 0);
-    }
+    __syncthreads();  // a previous pass may still be reading either buffer
+    issue(n_begin, 0);
     auto tile = [&](int n0, auto buf_c) __attribute__((always_inline)) {
       constexpr int buf = decltype(buf_c)::value;
-      if constexpr (PF == 2) {
-        // this wave's loads of tile n0 have landed; after the barrier everybody's have, and nobody
-        // reads the other buffer any more: the next tile goes there
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (n0 + kBN < blk_b) issue(n0 + kBN, buf ^ 1);
-      } else {
-        __syncthreads();
-        if (PF) stash(); else direct(n0);
-        __syncthreads();
-        if (PF && n0 + kBN < blk_b) fetch(n0 + kBN);
-      }
+      // this wave's loads of tile n0 have landed; after the barrier everybody's have, and nobody
+      // reads the other buffer any more: the next tile goes there
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (n0 + kBN < blk_b) issue(n0 + kBN, buf ^ 1);
       const uint8_t* const tk = fwd_smem + buf * SM::kBuf;
-      const uint8_t* const tv = tk + SM::kTileK;
+      const uint8_t* const tv = tk + SM::kTile;
       if (n0 >= w_bmax || n0 + kBN <= w_amin) return;  // nothing visible for this wave
 
       f32x16 st[NSB][2];
@@ -528,12 +519,9 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
         auto kread = [&](int f) {
           if constexpr (kAbsRd)
             kfr[f % RG] = as_bf16x8(lds_read128(krd[f >> 1] + buf * SM::kBuf + (f & 1) * 32 * RBK));
-          else if constexpr (PF == 2)
-            kfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                tk + (f & 1) * 32 * RBK + (rdk ^ ((f >> 1) * 32))));
           else
             kfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                &Ks[((f & 1) * 32 + col) * KS + g * 8 + (f >> 1) * 16]));
+                tk + (f & 1) * 32 * RBK + (rdk ^ ((f >> 1) * 32))));
         };
 #pragma unroll
         for (int f = 0; f < RG; ++f) kread(f);
@@ -616,14 +604,23 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
         constexpr int RG = SPX_FWD_RING;
         bf16x8 vfr[RG];
         auto vread = [&](int f) {
-          if constexpr (kAbsRd)
-            vfr[f % RG] = as_bf16x8(lds_read128(vrd[f / NDB] + buf * SM::kBuf + (f % NDB) * 32 * 128));
-          else if constexpr (PF == 2)
-            vfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                tv + (f % NDB) * 32 * 128 + (rdv ^ ((f / NDB) * 32))));
-          else
-            vfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                &Vs[((f % NDB) * 32 + col) * VS + (f / NDB) * 16 + 8 * g]));
+          if constexpr (!TR) {
+            if constexpr (kAbsRd)
+              vfr[f % RG] = as_bf16x8(lds_read128(vrd[f / NDB] + buf * SM::kBuf + (f % NDB) * 32 * 128));
+            else
+              vfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
+                  tv + (f % NDB) * 32 * 128 + (rdv ^ ((f / NDB) * 32))));
+            return;
+          }
+          i16x4 lo, hi;
+          if constexpr (kAbsRd) {
+            lo = lds_tr16(vrd0[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
+            hi = lds_tr16(vrd1[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
+          } else {
+            lo = lds_read_tr16(tv + (f / NDB) * 16 * RBK + (rt0 ^ ((f % NDB) * 64)));
+            hi = lds_read_tr16(tv + (f / NDB) * 16 * RBK + (rt1 ^ ((f % NDB) * 64)));
+          }
+          vfr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         };
 #pragma unroll
         for (int f = 0; f < RG; ++f) vread(f);
@@ -795,91 +792,92 @@ __device__ __forceinline__ void st_bf16s(uint16_t* p, const float (&v)[EPL]) {
   }
 }
 
-__global__ __launch_bounds__(256) void fill_zero_kernel(float* __restrict__ x, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) x[i] = 0.f;
-}
-
+// What the backward kernels read next to the operands, in one launch (five small ones took 4 us each whatever their
+// size; 512 rows of 32 heads of 64: 18 -> 6 us).  Sixteen lanes per (head, row), D / 16 consecutive elements each:
+//   qs[h][i]   bf16(q * scale * log2 e), row-major;
+//   delta      dO . O of the row (summed with DPP moves), [Hq][NQ];
+//   neg        -lse and -delta in rows of NQp (zero in the padding): C operands of the dK / dV score products;
+// and in the last blocks, one wave per 64-row query tile, the interval ends of its rows and their extremes:
+//   rows[4][NQp]  a1, b1, T + a2, T + b2 as the kernels compare them (empty where a class is absent or the row is padding)
+//   tb[tile][8]   [a1min, a1max, b1min, b1max, a2min, a2max, b2min, b2max]
 template <int D>
-__global__ __launch_bounds__(256) void attn_delta_kernel(const uint16_t* __restrict__ O,
-                                                         const uint16_t* __restrict__ dO, int NQ,
-                                                         int Hq, float* __restrict__ delta,
-                                                         const float* __restrict__ lse, int NQp,
-                                                         float* __restrict__ neg) {
-  // sixteen lanes per (row, head): D / 16 consecutive elements each, summed with DPP moves
-  constexpr int EPL = D / 16;
-  const int64_t n_rows = (int64_t)NQ * Hq;
-  const int64_t raw = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + ((threadIdx.x & 63) >> 4);
-  const int64_t row = raw < n_rows ? raw : n_rows - 1;  // = i * Hq + h
-  const int d0 = (threadIdx.x & 15) * EPL;
-  float a[EPL], b[EPL];
-  ld_bf16s<EPL>(O + row * D + d0, a);
-  ld_bf16s<EPL>(dO + row * D + d0, b);
-  float acc = 0.f;
+__global__ __launch_bounds__(256) void attn_bwd_prep_kernel(AttnParams p, const uint16_t* __restrict__ O,
+                                                            const uint16_t* __restrict__ dO,
+                                                            const float* __restrict__ lse, int NQp, int row_blocks,
+                                                            uint16_t* __restrict__ qs, float* __restrict__ delta,
+                                                            float* __restrict__ neg, int32_t* __restrict__ tb,
+                                                            int32_t* __restrict__ rows) {
+  if ((int)blockIdx.x >= row_blocks) {
+    const int tile = ((int)blockIdx.x - row_blocks) * 4 + (threadIdx.x >> 6);
+    const int r = tile * 64 + (threadIdx.x & 63);
+    if (tile * 64 >= NQp) return;
+    const bool ok = r < p.NQ;
+    const int a1 = ok ? p.a1[r] : 0x7fffffff;
+    const int b1 = ok ? (p.b1 ? p.b1[r] : r + 1) : 0;
+    const int a2 = (ok && p.a2) ? p.T + p.a2[r] : 0x7fffffff;
+    const int b2 = (ok && p.a2) ? p.T + p.b2[r] : 0;
+    rows[r] = a1; rows[NQp + r] = b1; rows[2 * (int64_t)NQp + r] = a2; rows[3 * (int64_t)NQp + r] = b2;
+    const int v[8] = {wave_min_i(a1), wave_max_i(a1), wave_min_i(b1), wave_max_i(b1),
+                      wave_min_i(a2), wave_max_i(a2), wave_min_i(b2), wave_max_i(b2)};
+    if ((threadIdx.x & 63) == 0 && tile * 64 < p.NQ) {
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) acc = fmaf(a[e], b[e], acc);
+      for (int k = 0; k < 8; ++k) tb[tile * 8 + k] = v[k];
+    }
+    return;
+  }
+  constexpr int EPL = D / 16;
+  const int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);  // = h * NQp + i
+  const int h = (int)(item / NQp), i = (int)(item % NQp);
+  if (h >= p.Hq) return;  // (whole groups of sixteen lanes)
+  const int d0 = (threadIdx.x & 15) * EPL;
+  const bool live = i < p.NQ;
+  float acc = 0.f;
+  if (live) {
+    const int64_t row = (int64_t)i * p.Hq + h;
+    float a[EPL], b[EPL], q[EPL];
+    ld_bf16s<EPL>(O + row * D + d0, a);
+    ld_bf16s<EPL>(dO + row * D + d0, b);
+    ld_bf16s<EPL>(p.Q + (int64_t)h * p.q_hs + (int64_t)i * D + d0, q);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      acc = fmaf(a[e], b[e], acc);
+      q[e] *= p.scale_log2e;  // (the same rounded values as scale_bf16x8 gives)
+    }
+    st_bf16s<EPL>(qs + ((int64_t)h * p.NQ + i) * D + d0, q);
+  }
   acc = row16_sum(acc);
-  if ((threadIdx.x & 15) == 0 && raw < n_rows) {
-    const int64_t hh = row % Hq, i = row / Hq;
-    delta[hh * NQ + i] = acc;
-    // -lse and -delta in rows of NQp (the padding stays zero: see the launcher), the C operands of the
-    // wave-specialised dK/dV kernel's score products
-    neg[hh * NQp + i] = -lse[hh * NQ + i];
-    neg[((int64_t)Hq + hh) * NQp + i] = -acc;
+  if ((threadIdx.x & 15) == 0) {
+    if (live) delta[(int64_t)h * p.NQ + i] = acc;
+    neg[item] = live ? -lse[(int64_t)h * p.NQ + i] : 0.f;
+    neg[(int64_t)p.Hq * NQp + item] = live ? -acc : 0.f;
   }
 }
 
 // dQ: same tiling as the forward.
 //   P^T = exp2(S'^T - lse), dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
-// PF: how a key tile reaches LDS: 0 through registers at the point of use, 1 through registers one tile
-// ahead, 3 global -> LDS directly into the other of two buffers, with tiles of 32 instead of 64 keys so
-// that two buffers of the three tiles (K, V, K^T) fit beside a second workgroup (see FwdSmem).
-// Four 16-bit values per lane from LDS, transposed inside every group of 16 lanes: lane 4u + w of
-// a group receives, as element j, element w of the 8 bytes that lane 4j + u of the group points at.
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) i16x4*)(uintptr_t)(uint32_t)(uintptr_t)(
-          (__attribute__((address_space(3))) const uint8_t*)p));
-}
-
-template <int D, int NW, int PF>
+template <int D, int NW>
 struct DqSmem {
-  // mode 4: only the row-major K and V tiles, 64 keys each; the K^T fragments of the dQ product come
+  // the row-major K and V tiles, 64 keys each; the K^T fragments of the dQ product come
   // out of the K tile through transposing LDS reads
-  static constexpr int TB = PF == 3 ? 32 : (PF == 4 ? 64 : kBN);     // keys per tile
-  static constexpr int KS = D + kKPad, VS = kBN + kVPad;
-  static constexpr int kTileK = TB * D * 2, kTileT = PF == 4 ? 0 : D * TB * 2;  // modes 3, 4: unpadded, swizzled
-  static constexpr int kBuf = 2 * kTileK + kTileT;
+  static constexpr int kTileK = kBN * D * 2;
+  static constexpr int kBuf = 2 * kTileK;
   static constexpr int kDiag = NW * 2 * 32 * D * 2;  // K and V rows of 32 queries per wave (TTT diagonal keys)
-  static constexpr int kTiles0 = PF >= 3 ? 2 * kBuf : (2 * kBN * KS + D * VS) * 2;
-  static constexpr int kTiles = kTiles0 > kDiag ? kTiles0 : kDiag;
+  static constexpr int kTiles = 2 * kBuf > kDiag ? 2 * kBuf : kDiag;
   static constexpr int kBytes = kTiles + 4 * NW * (int)sizeof(int);
 };
 
-template <int D, int NSB, int NW, int PF>
+template <int D, int NSB, int NW>
 __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_dq_kernel(
-    AttnParams p, const uint16_t* __restrict__ dO, const uint16_t* __restrict__ Kt,
-    const float* __restrict__ LSE, const float* __restrict__ Delta, uint16_t* __restrict__ dQ,
+    AttnParams p, const uint16_t* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ Delta, uint16_t* __restrict__ dQ,
     int64_t dq_hs) {
-  using SM = DqSmem<D, NW, PF>;
-  constexpr bool kDma = PF >= 3;
-  constexpr bool kTR = PF == 4;
-  constexpr int TB = SM::TB;
-  constexpr int KS = SM::KS;
-  constexpr int VS = SM::VS;
+  using SM = DqSmem<D, NW>;
+  constexpr int TB = kBN;
   constexpr int NKK = D / 16;
   constexpr int NDB = D / 32;
-  constexpr int NT = 64 * NW;
-  constexpr int CPT = (kBN * D / 8) / NT;
   constexpr int BMW = 32 * NSB;
   constexpr int BM = NW * BMW;
 
   extern __shared__ __attribute__((aligned(16))) uint8_t dq_smem[];
-  uint16_t* const Ks = reinterpret_cast<uint16_t*>(dq_smem);
-  uint16_t* const Vn = Ks + kBN * KS;
-  uint16_t* const Kts = Vn + kBN * KS;
   int* const red = reinterpret_cast<int*>(dq_smem + SM::kTiles);
 
   const int group = p.Hq / p.Hkv;
@@ -932,95 +930,31 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
 
   const uint16_t* Kh = p.K + (int64_t)kvh * p.k_hs;
   const uint16_t* Vh = p.V + (int64_t)kvh * p.v_hs;
-  const uint16_t* Kth = Kt + (int64_t)kvh * D * p.NKVp;
   const int last_row = p.NKV - 1;
 
-  u32x4 kreg[CPT], vreg[CPT], treg[CPT];
-  auto fetch = [&](int n0) {
-    // offsets recomputed per tile on purpose (see the dK/dV kernel): kept live through the loop they spill
-    // at head_dim 256, and a spill reload waits for the prefetch issued here
-    int tid_v = tid;
-    if (SPX_DKV_REMAT) asm volatile("" : "+v"(tid_v));
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid_v + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      const int kr = min(n0 + krow, last_row);
-      kreg[n] = *reinterpret_cast<const u32x4*>(Kh + (int64_t)kr * D + kcol);
-      vreg[n] = *reinterpret_cast<const u32x4*>(Vh + (int64_t)kr * D + kcol);
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      treg[n] = *reinterpret_cast<const u32x4*>(Kth + (int64_t)vd * p.NKVp + n0 + vcol);
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      *reinterpret_cast<u32x4*>(&Ks[krow * KS + kcol]) = kreg[n];
-      *reinterpret_cast<u32x4*>(&Vn[krow * KS + kcol]) = vreg[n];
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      *reinterpret_cast<u32x4*>(&Kts[vd * VS + vcol]) = treg[n];
-    }
-  };
-
-  auto direct = [&](int n0) {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int c = tid + NT * n;
-      const int krow = c / (D / 8), kcol = (c % (D / 8)) * 8;
-      const int kr = min(n0 + krow, last_row);
-      *reinterpret_cast<u32x4*>(&Ks[krow * KS + kcol]) =
-          *reinterpret_cast<const u32x4*>(Kh + (int64_t)kr * D + kcol);
-      *reinterpret_cast<u32x4*>(&Vn[krow * KS + kcol]) =
-          *reinterpret_cast<const u32x4*>(Vh + (int64_t)kr * D + kcol);
-      const int vd = c >> 3, vcol = (c & 7) * 8;
-      const u32x4 t = *reinterpret_cast<const u32x4*>(Kth + (int64_t)vd * p.NKVp + n0 + vcol);
-      *reinterpret_cast<u32x4*>(&Kts[vd * VS + vcol]) = t;
-    }
-  };
-
-  // ---- mode 3: the three tiles as 1 KB wave loads global -> LDS (chunk c of row r in slot c ^ swz(r))
+  // ---- the two tiles as 1 KB wave loads global -> LDS (chunk c of row r in slot c ^ swz(r))
   constexpr int RBK = D * 2, CKK = RBK / 16;   // bytes / 16-byte chunks per row of K and V
-  constexpr int RBT = TB * 2, CKT = RBT / 16;  // ... of K^T
-  constexpr int LPK = (TB * RBK / 1024) / NW, LPT = (D * RBT / 1024) / NW;
-  auto swz_k = [](int r) {
-    // (transposing reads touch 4 + 4 rows x 64 bytes: those rows must fall into different 64-byte bank groups)
-    if (kTR) return CKK == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3);
-    return CKK == 8 ? (r >> 1) & 7 : r & 15;
-  };
-  auto swz_t = [](int r) { return CKT == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  constexpr int LPK = (TB * RBK / 1024) / NW;
+  // (transposing reads touch 4 + 4 rows x 64 bytes: those rows must fall into different 64-byte bank groups)
+  auto swz_k = [](int r) { return CKK == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3); };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dq_smem;
-  u32x4 kres, vres, tres;
-  if constexpr (kDma) {
-    static_assert(!kDma || (LPK >= 1 && LPT >= 1), "a tile is at least one 1 KB load per wave");
-    kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
-    vres = make_rsrc(Vh, (uint32_t)((int64_t)p.NKV * RBK));
-    tres = make_rsrc(Kth, (uint32_t)((int64_t)D * p.NKVp * 2));
-  }
+  const u32x4 kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
+  const u32x4 vres = make_rsrc(Vh, (uint32_t)((int64_t)p.NKV * RBK));
   auto issue = [&](int n0, int b) __attribute__((always_inline)) {
-    if constexpr (kDma) {
-      int lane_v = lane;
-      if (SPX_DKV_REMAT) asm volatile("" : "+v"(lane_v));  // offsets recomputed per tile, not kept live
-      const uint32_t kb0 = lds0 + b * SM::kBuf + wave * LPK * 1024;
+    int lane_v = lane;
+    asm volatile("" : "+v"(lane_v));  // offsets recomputed per tile, not kept live
+    const uint32_t kb0 = lds0 + b * SM::kBuf + wave * LPK * 1024;
 #pragma unroll
-      for (int j = 0; j < LPK; ++j) {
-        const int r = (wave * LPK + j) * (1024 / RBK) + lane_v / CKK;
-        const int off = min(n0 + r, last_row) * RBK + ((lane_v % CKK) ^ swz_k(r)) * 16;
-        load_to_lds16<0>(kres, kb0 + j * 1024, off, 0);
-        load_to_lds16<0>(vres, kb0 + SM::kTileK + j * 1024, off, 0);
-      }
-      const uint32_t tb0 = lds0 + b * SM::kBuf + 2 * SM::kTileK + wave * LPT * 1024;
-#pragma unroll
-      for (int j = 0; j < (kTR ? 0 : LPT); ++j) {
-        const int r = (wave * LPT + j) * (1024 / RBT) + lane_v / CKT;
-        load_to_lds16<0>(tres, tb0 + j * 1024, r * p.NKVp * 2 + ((lane_v % CKT) ^ swz_t(r)) * 16, n0 * 2);
-      }
+    for (int j = 0; j < LPK; ++j) {
+      const int r = (wave * LPK + j) * (1024 / RBK) + lane_v / CKK;
+      const int off = min(n0 + r, last_row) * RBK + ((lane_v % CKK) ^ swz_k(r)) * 16;
+      load_to_lds16<0>(kres, kb0 + j * 1024, off, 0);
+      load_to_lds16<0>(vres, kb0 + SM::kTileK + j * 1024, off, 0);
     }
   };
   const int rdk = col * RBK + ((g ^ swz_k(col)) * 16);
-  const int rdt = col * RBT + ((g ^ swz_t(col)) * 16);
-  // transposing reads (see the dK/dV kernel): rows 4 (G >> 1) + (s >> 2) (+ 8) of a 16-key step
+  // transposing reads: lane s of 16-lane group G points at row 4 (G >> 1) + (s >> 2) (+ 8 for the second read) of a
+  // 16-key step, bytes 8 (s & 3) of the 64-byte block 32 db + 16 (G & 1)
   const int tG = lane >> 4, ts = lane & 15;
   const int trow = 4 * (tG >> 1) + (ts >> 2);
   const int tcl = 2 * (tG & 1) + ((ts & 3) >> 1);
@@ -1031,23 +965,13 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
                       int w_bmin, int w_bmax, int blk_a, int blk_b) {
     if (blk_b <= blk_a) return;
     const int n_begin = (blk_a / TB) * TB;
-    if (PF == 1) fetch(n_begin);
     int buf = 0;
-    if constexpr (kDma) {
-      __syncthreads();  // a previous pass may still be reading either buffer
-      issue(n_begin, 0);
-    }
+    __syncthreads();  // a previous pass may still be reading either buffer
+    issue(n_begin, 0);
     for (int n0 = n_begin; n0 < blk_b; n0 += TB) {
-      if constexpr (kDma) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (n0 + TB < blk_b) issue(n0 + TB, buf ^ 1);
-      } else {
-        __syncthreads();
-        if (PF) stash(); else direct(n0);
-        __syncthreads();
-        if (PF && n0 + kBN < blk_b) fetch(n0 + kBN);
-      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (n0 + TB < blk_b) issue(n0 + TB, buf ^ 1);
       const uint8_t* const tile = dq_smem + buf * SM::kBuf;
       buf ^= 1;
       if (n0 >= w_bmax || n0 + TB <= w_amin) continue;
@@ -1056,7 +980,7 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb) {
         // the 32-key halves of the tile one after the other: 32 score registers live
-#pragma unroll(kTR && D > 128 ? 1 : TB / 32)
+#pragma unroll(D > 128 ? 1 : TB / 32)
         for (int kb = 0; kb < TB / 32; ++kb) {
           f32x16 st, dp;
           // K and V fragments alternate through a ring of four registers (fragment 2 kk is
@@ -1066,14 +990,8 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
             constexpr int NF = 2 * NKK;
             bf16x8 fr[4];
             auto fread = [&](int f) {
-              if constexpr (kDma) {
-                fr[f & 3] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                    tile + ((f & 1) ? SM::kTileK : 0) + kb * 32 * RBK + (rdk ^ ((f >> 1) * 32))));
-              } else {
-                const uint16_t* base = (f & 1) ? Vn : Ks;
-                fr[f & 3] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                    &base[(kb * 32 + col) * KS + g * 8 + (f >> 1) * 16]));
-              }
+              fr[f & 3] = as_bf16x8(*reinterpret_cast<const u32x4*>(
+                  tile + ((f & 1) ? SM::kTileK : 0) + kb * 32 * RBK + (rdk ^ ((f >> 1) * 32))));
             };
 #pragma unroll
             for (int f = 0; f < 4; ++f) fread(f);
@@ -1109,17 +1027,10 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
             constexpr int NF = 2 * NDB;
             bf16x8 fr[4];
             auto fread = [&](int f) {
-              if constexpr (kTR) {
-                const uint8_t* base = tile + (kb * 32 + (f / NDB) * 16) * RBK;
-                const i16x4 lo = lds_read_tr16(base + (rt0 ^ ((f % NDB) * 64)));
-                const i16x4 hi = lds_read_tr16(base + (rt1 ^ ((f % NDB) * 64)));
-                fr[f & 3] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-              } else if constexpr (kDma)
-                fr[f & 3] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                    tile + 2 * SM::kTileK + (f % NDB) * 32 * RBT + (rdt ^ ((kb * 2 + f / NDB) * 32))));
-              else
-                fr[f & 3] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                    &Kts[((f % NDB) * 32 + col) * VS + (kb * 2 + f / NDB) * 16 + 8 * g]));
+              const uint8_t* base = tile + (kb * 32 + (f / NDB) * 16) * RBK;
+              const i16x4 lo = lds_read_tr16(base + (rt0 ^ ((f % NDB) * 64)));
+              const i16x4 hi = lds_read_tr16(base + (rt1 ^ ((f % NDB) * 64)));
+              fr[f & 3] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             };
 #pragma unroll
             for (int f = 0; f < 4 && f < NF; ++f) fread(f);
@@ -1213,959 +1124,14 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
   }
 }
 
-// per 64-row query tile: min / max of the interval ends of both classes (for the dK/dV
-// tile loop): [a1min, a1max, b1min, b1max, a2min, a2max, b2min, b2max]
-// rows[4][NQp] (NQp a multiple of 64): the interval ends of every row as the kernels compare them
-// (a1, b1, T + a2, T + b2; an empty interval where a class is absent or the row is padding)
-__global__ __launch_bounds__(64) void attn_tile_bounds_kernel(AttnParams p, int32_t* __restrict__ tb,
-                                                              int NQp, int32_t* __restrict__ rows) {
-  const int tile = blockIdx.x;
-  const int r = tile * 64 + threadIdx.x;
-  const bool ok = r < p.NQ;
-  const int a1 = ok ? p.a1[r] : 0x7fffffff;
-  const int b1 = ok ? (p.b1 ? p.b1[r] : r + 1) : 0;
-  const int a2 = (ok && p.a2) ? p.T + p.a2[r] : 0x7fffffff;
-  const int b2 = (ok && p.a2) ? p.T + p.b2[r] : 0;
-  if (r < NQp) {
-    rows[r] = a1; rows[NQp + r] = b1; rows[2 * (int64_t)NQp + r] = a2; rows[3 * (int64_t)NQp + r] = b2;
-  }
-  const int v[8] = {wave_min_i(a1), wave_max_i(a1), wave_min_i(b1), wave_max_i(b1),
-                    wave_min_i(a2), wave_max_i(a2), wave_min_i(b2), wave_max_i(b2)};
-  if (threadIdx.x == 0 && tile * 64 < p.NQ) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) tb[tile * 8 + k] = v[k];
-  }
-}
+}  // namespace spx
+#include "attn_dkv.h"
+namespace spx {
 
-// dK / dV of the tiled keys: one workgroup = 128 keys x ONE query head (a wave owns 32
-// keys: lane column = key), looping over the 64-row query tiles that can see the block.
-// Scores are produced in the S = Q K^T orientation so that a lane holds one KEY:
-//   dV^T += dO^T P,   dK^T += Q^T dS,   dS = P (dO V^T - delta)
-// The per-head results go to fp32 partial buffers that attn_dkv_reduce_kernel sums over
-// the heads of a group (fixed order: deterministic, no atomics).
-// PASS 0 computes dK and dV together; PASS 1 only dV, PASS 2 only dK (head_dim 256: the two
-// accumulator sets and both operand fragments do not fit the register file together, so
-// the kernel is launched once per pass and the scores are recomputed).
-#define SPX_DKV_XCD 1
-// PF: how the query tiles reach LDS (see FwdSmem): 0 at the point of use, 1 through registers one
-// tile ahead, 2 global -> LDS into the other of two buffers, 3 the same with tiles of 32 instead of 64
-// query rows.  A buffer holds the tiles the pass multiplies with: Q always, dO and Q^T for dK, dO^T for
-// dV.  At head_dim 256 two buffers of 64-row tiles fit the 160 KB of LDS only for the dV pass; with
-// 32-row tiles all four fit, the register staging is gone and dK and dV come out of ONE pass.
-// 4: like 2, but only the row-major Q and dO tiles are loaded: the A operands of the accumulating
-// products (Q^T, dO^T fragments) come out of them through the transposing LDS read of gfx950
-// (ds_read_b64_tr_b16), so two buffers of 64-row tiles fit at head_dim 256 as well, a step is 64
-// rows long and half as many loads are issued per row.
-template <int D, int PASS, int QT = 64, bool TR = false>
-struct DkvSmem {
-  static constexpr bool kDoV = PASS != 2, kDoK = PASS != 1;
-  static constexpr int kTileR = QT * D * 2, kTileT = TR ? 0 : D * QT * 2;  // Q / dO and Q^T / dO^T tiles, unpadded
-  static constexpr int kOffdO = kTileR;
-  static constexpr int kOffQt = ((kDoK || TR) ? 2 : 1) * kTileR;
-  static constexpr int kOffdOt = kOffQt + (kDoK ? kTileT : 0);
-  static constexpr int kBuf = kOffdOt + (kDoV ? kTileT : 0);
-  static constexpr int kSmall = 6 * 64 * 4;                     // lse, delta, a1, b1, a2, b2 of 64 rows
-  static constexpr int kBytesDma = 2 * kBuf + 2 * kSmall;
-  static constexpr int kBytes = (2 * 64 * (D + kKPad) + 2 * D * (64 + kVPad)) * 2 + kSmall;
-};
-
-// operand fragments in flight per product in the dK/dV kernel (one wave per SIMD: nothing else
-// hides the latency of its LDS reads)
-#define SPX_DKV_RING 8
-template <int D, int NW, int PF, int PASS>
-__global__ __launch_bounds__(64 * NW, SPX_DKV_MINB) void attn_bwd_dkv_kernel(
-    AttnParams p, const uint16_t* __restrict__ dO, const uint16_t* __restrict__ Qt,
-    const uint16_t* __restrict__ dOt, int NQp, const float* __restrict__ LSE,
-    const float* __restrict__ Delta, const int32_t* __restrict__ tile_bounds,
-    float* __restrict__ dKp, float* __restrict__ dVp) {
-  constexpr int QS = D + kKPad;
-  constexpr int TS = 64 + kVPad;
-  constexpr int NKK = D / 16;
-  constexpr int NDB = D / 32;
-  constexpr int NT = 64 * NW;
-  constexpr int KB = 32 * NW;  // keys per workgroup
-  constexpr int CPT = (64 * D / 8) / NT;
-
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  uint16_t* Qs = smem;                 // [64][QS]
-  uint16_t* dOs = Qs + 64 * QS;        // [64][QS]
-  uint16_t* Qts = dOs + 64 * QS;       // [D][TS]
-  uint16_t* dOts = Qts + D * TS;       // [D][TS]
-  constexpr bool kDma = PF >= 2;
-  constexpr bool kTR = PF == 4;                  // transposed operands by transposing LDS reads
-  constexpr int QT = PF == 3 ? 32 : 64;          // query rows per LDS tile
-  constexpr int NQB = QT / 32, NSUB = 64 / QT;   // 32-row halves per tile, tiles per 64-row step
-  using SM = DkvSmem<D, PASS, QT, kTR>;
-  static_assert(!kTR || PASS == 0, "the transposing-read mode computes both gradients");
-  static_assert(!kDma || SM::kBytesDma <= 160 * 1024, "two buffers of this pass's tiles do not fit in LDS");
-  uint8_t* const sm8 = reinterpret_cast<uint8_t*>(smem);
-  float* lse_s = reinterpret_cast<float*>(kDma ? sm8 + 2 * SM::kBuf : sm8 + (2 * 64 * QS + 2 * D * TS) * 2);  // [64]
-  float* delta_s = lse_s + 64;                               // [64]
-  int* a1_s = reinterpret_cast<int*>(delta_s + 64);          // [64] each
-  int* b1_s = a1_s + 64;
-  int* a2_s = b1_s + 64;
-  int* b2_s = a2_s + 64;
-
-  // Workgroups go to the eight XCDs round robin.  The query-side tiles a workgroup streams belong to
-  // its query head, so the workgroups that share an XCD (and its L2) at a time get the SAME head and
-  // consecutive key blocks: neighbours in that order read the same tile two steps apart.
-  // Heavy key blocks first: under a causal mask the EARLY key blocks are seen by most rows.
-  int h, kb_idx;
-  if (SPX_DKV_XCD && p.Hq % 8 == 0) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, n_kb = gridDim.x / p.Hq;
-    h = xcd + 8 * (slot / n_kb);
-    kb_idx = slot % n_kb;
-  } else {
-    h = blockIdx.x % p.Hq;
-    kb_idx = blockIdx.x / p.Hq;
-  }
-  const int kvh = h / (p.Hq / p.Hkv);
-  const int n0 = kb_idx * KB;
-  const int key_last = min(n0 + KB - 1, p.NKV - 1);
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, col = lane & 31;
-  const int cw = n0 + wave * 32;
-  const int c = cw + col;
-  const int cc = c < p.NKV ? c : p.NKV - 1;
-
-  constexpr bool kDoV = PASS != 2, kDoK = PASS != 1;
-  constexpr int NVF = kDoK ? NKK : 1;                    // V fragments feed dP, a dK-only term
-  constexpr int NAK = kDoK ? NDB : 1, NAV = kDoV ? NDB : 1;
-  bf16x8 kf[NKK], vf[NVF];
-  {
-    const uint16_t* krow = p.K + (int64_t)kvh * p.k_hs + (int64_t)cc * D + g * 8;
-    const uint16_t* vrow = p.V + (int64_t)kvh * p.v_hs + (int64_t)cc * D + g * 8;
-#pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
-      kf[kk] = as_bf16x8(*reinterpret_cast<const u32x4*>(krow + kk * 16));
-      if (kDoK) vf[kk % NVF] = as_bf16x8(*reinterpret_cast<const u32x4*>(vrow + kk * 16));
-    }
-  }
-  f32x16 acc_dk[NAK], acc_dv[NAV];
-#pragma unroll
-  for (int db = 0; db < NAK; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc_dk[db][r] = 0.f;
-#pragma unroll
-  for (int db = 0; db < NAV; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc_dv[db][r] = 0.f;
-
-  const uint16_t* Qh = p.Q + (int64_t)h * p.q_hs;
-  const uint16_t* Qth = Qt + (int64_t)h * D * NQp;
-  const uint16_t* dOth = dOt + (int64_t)h * D * NQp;
-  const int n_qt = (p.NQ + 63) / 64;
-
-  u32x4 qreg[CPT], dreg[CPT], qtreg[CPT], dtreg[CPT];
-  float lse_r = 0.f, delta_r = 0.f;
-  int a1_r = 0, b1_r = 0, a2_r = 0, b2_r = 0;
-  auto visible = [&](int qt) {
-    const int ta1 = tile_bounds[qt * 8 + 0], tb1 = tile_bounds[qt * 8 + 3];
-    const int ta2 = tile_bounds[qt * 8 + 4], tb2 = tile_bounds[qt * 8 + 7];
-    return (ta1 <= key_last && tb1 > n0) || (ta2 <= key_last && tb2 > n0);
-  };
-  // every row of the tile sees every key of this block: no per-element interval test
-  auto fully_visible = [&](int qt) {
-    return (tile_bounds[qt * 8 + 1] <= n0 && tile_bounds[qt * 8 + 2] >= n0 + KB) ||
-           (tile_bounds[qt * 8 + 5] <= n0 && tile_bounds[qt * 8 + 6] >= n0 + KB);
-  };
-  // the per-row scalars of a query tile: wave 0 loads them into registers ...
-  auto small_fetch = [&](int mq) {
-    if (tid < 64) {
-      const int ir = mq + tid;
-      const bool ok = ir < p.NQ;
-      lse_r = ok ? -LSE[(int64_t)h * p.NQ + ir] : 0.f;    // negated: they are MFMA C operands
-      delta_r = ok ? -Delta[(int64_t)h * p.NQ + ir] : 0.f;
-      a1_r = ok ? p.a1[ir] : 0x7fffffff;
-      b1_r = ok ? (p.b1 ? p.b1[ir] : ir + 1) : 0;
-      a2_r = (ok && p.a2) ? p.T + p.a2[ir] : 0x7fffffff;
-      b2_r = (ok && p.a2) ? p.T + p.b2[ir] : 0;
-    }
-  };
-  // ... and writes them to LDS (set `b` of the six arrays: only the two-buffer mode has a second one)
-  auto small_stash = [&](int b) {
-    if (tid < 64) {
-      const int o = b * (SM::kSmall / 4);
-      lse_s[o + tid] = lse_r; delta_s[o + tid] = delta_r;
-      a1_s[o + tid] = a1_r; b1_s[o + tid] = b1_r; a2_s[o + tid] = a2_r; b2_s[o + tid] = b2_r;
-    }
-  };
-  auto fetch = [&](int mq) {
-    // The per-load row / column offsets are recomputed here on purpose.  Hoisted out of the tile loop they
-    // stay live through it, and at head_dim 256 that is what spills; a spill reload inside the loop waits
-    // for every older vector-memory operation, i.e. for the prefetch this function has just issued.
-    int tid_v = tid;
-    if (SPX_DKV_REMAT) asm volatile("" : "+v"(tid_v));
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int ch = tid_v + NT * n;
-      const int qr = ch / (D / 8), qc = (ch % (D / 8)) * 8;
-      const int ir = min(mq + qr, p.NQ - 1);
-      qreg[n] = *reinterpret_cast<const u32x4*>(Qh + (int64_t)ir * D + qc);
-      if (kDoK) dreg[n] = *reinterpret_cast<const u32x4*>(dO + ((int64_t)ir * p.Hq + h) * D + qc);
-      const int td = ch >> 3, tc = (ch & 7) * 8;
-      if (kDoK) qtreg[n] = *reinterpret_cast<const u32x4*>(Qth + (int64_t)td * NQp + mq + tc);
-      if (kDoV) dtreg[n] = *reinterpret_cast<const u32x4*>(dOth + (int64_t)td * NQp + mq + tc);
-    }
-    small_fetch(mq);
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int ch = tid + NT * n;
-      const int qr = ch / (D / 8), qc = (ch % (D / 8)) * 8;
-      *reinterpret_cast<u32x4*>(&Qs[qr * QS + qc]) = qreg[n];
-      if (kDoK) *reinterpret_cast<u32x4*>(&dOs[qr * QS + qc]) = dreg[n];
-      const int td = ch >> 3, tc = (ch & 7) * 8;
-      if (kDoK) *reinterpret_cast<u32x4*>(&Qts[td * TS + tc]) = qtreg[n];
-      if (kDoV) *reinterpret_cast<u32x4*>(&dOts[td * TS + tc]) = dtreg[n];
-    }
-    small_stash(0);
-  };
-
-  auto direct = [&](int mq) {
-#pragma unroll
-    for (int n = 0; n < CPT; ++n) {
-      const int ch = tid + NT * n;
-      const int qr = ch / (D / 8), qc = (ch % (D / 8)) * 8;
-      const int ir = min(mq + qr, p.NQ - 1);
-      // only the tiles this pass multiplies with: Q always (scores), dO and Q^T for dK,
-      // dO^T for dV
-      *reinterpret_cast<u32x4*>(&Qs[qr * QS + qc]) =
-          *reinterpret_cast<const u32x4*>(Qh + (int64_t)ir * D + qc);
-      if (kDoK)
-        *reinterpret_cast<u32x4*>(&dOs[qr * QS + qc]) =
-            *reinterpret_cast<const u32x4*>(dO + ((int64_t)ir * p.Hq + h) * D + qc);
-      const int td = ch >> 3, tc = (ch & 7) * 8;
-      if (kDoK)
-        *reinterpret_cast<u32x4*>(&Qts[td * TS + tc]) =
-            *reinterpret_cast<const u32x4*>(Qth + (int64_t)td * NQp + mq + tc);
-      if (kDoV)
-        *reinterpret_cast<u32x4*>(&dOts[td * TS + tc]) =
-            *reinterpret_cast<const u32x4*>(dOth + (int64_t)td * NQp + mq + tc);
-    }
-    if (tid < 64) {
-      const int ir = mq + tid;
-      const bool ok = ir < p.NQ;
-      lse_s[tid] = ok ? -LSE[(int64_t)h * p.NQ + ir] : 0.f;
-      delta_s[tid] = ok ? -Delta[(int64_t)h * p.NQ + ir] : 0.f;
-      a1_s[tid] = ok ? p.a1[ir] : 0x7fffffff;
-      b1_s[tid] = ok ? (p.b1 ? p.b1[ir] : ir + 1) : 0;
-      a2_s[tid] = (ok && p.a2) ? p.T + p.a2[ir] : 0x7fffffff;
-      b2_s[tid] = (ok && p.a2) ? p.T + p.b2[ir] : 0;
-    }
-  };
-
-  // ---- two-buffer modes: the tiles as 1 KB wave loads global -> LDS; chunk c of row r lives in
-  // slot c ^ swz(r) (conflict-free fragment reads without padding)
-  constexpr int RBQ = D * 2, CKQ = RBQ / 16;   // bytes / 16-byte chunks per row of Q and dO
-  constexpr int RBT = QT * 2, CKT = RBT / 16;  // ... of Q^T and dO^T
-  constexpr int LPR = (QT * RBQ / 1024) / NW, LPT = (D * RBT / 1024) / NW;  // wave loads per wave and tile
-  // (with transposing reads the rows of a 4 + 4 row group must also fall into different 64-byte bank
-  // groups: the row's two low bits go to the chunk index's bits 2 - 3)
-  auto swz_r = [](int r) {
-    if (kTR) return CKQ == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3);
-    return CKQ == 8 ? (r >> 1) & 7 : r & 15;
-  };
-  auto swz_t = [](int r) { return CKT == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)sm8;
-  u32x4 qres, dres, qtres, dtres;
-  if constexpr (kDma) {
-    qres = make_rsrc(Qh, (uint32_t)((int64_t)p.NQ * RBQ));
-    dres = make_rsrc(dO + (int64_t)h * D, (uint32_t)((((int64_t)p.NQ - 1) * p.Hq * D + D) * 2));
-    qtres = make_rsrc(Qth, (uint32_t)((int64_t)D * NQp * 2));
-    dtres = make_rsrc(dOth, (uint32_t)((int64_t)D * NQp * 2));
-  }
-  auto issue = [&](int mq, int b) __attribute__((always_inline)) {
-    if constexpr (kDma) {
-      // per-load offsets recomputed here on purpose: hoisted out of the tile loop they cost registers that
-      // the two-workgroups-per-CU build does not have
-      int lane_v = lane;
-      if (SPX_DKV_REMAT) asm volatile("" : "+v"(lane_v));
-      const uint32_t rb = lds0 + b * SM::kBuf + wave * LPR * 1024;
-#pragma unroll
-      for (int j = 0; j < LPR; ++j) {
-        const int r = (wave * LPR + j) * (1024 / RBQ) + lane_v / CKQ;
-        const int cofs = ((lane_v % CKQ) ^ swz_r(r)) * 16;
-        const int ir = min(mq + r, p.NQ - 1);
-        load_to_lds16<0>(qres, rb + j * 1024, ir * RBQ + cofs, 0);
-        if (kDoK || kTR) load_to_lds16<0>(dres, rb + SM::kOffdO + j * 1024, ir * (p.Hq * RBQ) + cofs, 0);
-      }
-      const uint32_t tb2 = lds0 + b * SM::kBuf + wave * LPT * 1024;
-#pragma unroll
-      for (int j = 0; j < (kTR ? 0 : LPT); ++j) {
-        const int r = (wave * LPT + j) * (1024 / RBT) + lane_v / CKT;
-        const int tofs = r * NQp * 2 + ((lane_v % CKT) ^ swz_t(r)) * 16;
-        if (kDoK) load_to_lds16<0>(qtres, tb2 + SM::kOffQt + j * 1024, tofs, mq * 2);
-        if (kDoV) load_to_lds16<0>(dtres, tb2 + SM::kOffdOt + j * 1024, tofs, mq * 2);
-      }
-    }
-  };
-  const int rdr = col * RBQ + ((g ^ swz_r(col)) * 16);
-  const int rdt = col * RBT + ((g ^ swz_t(col)) * 16);
-  // transposing reads: lane s of 16-lane group G points at row 4 (G >> 1) + (s >> 2) (+ 8 for the
-  // second read) of a 16-row k step, bytes 8 (s & 3) of the 64-byte block 32 db + 16 (G & 1): the k
-  // index order of the P / dS operands (rows 4 g .. 4 g + 3, then 8 + 4 g .. 8 + 4 g + 3)
-  const int tG = lane >> 4, ts = lane & 15;
-  const int trow = 4 * (tG >> 1) + (ts >> 2);
-  const int tcl = 2 * (tG & 1) + ((ts & 3) >> 1);
-  const int rt0 = trow * RBQ + ((tcl ^ swz_r(trow)) * 16) + (ts & 1) * 8;
-  const int rt1 = (trow + 8) * RBQ + ((tcl ^ swz_r(trow + 8)) * 16) + (ts & 1) * 8;
-  const float* const lse_s0 = lse_s;
-  const uint8_t* tile = sm8;
-  int buf = 0;
-
-  // (walking the tiles from the last one down, so that every workgroup of a head reads the same tile at
-  // the same time, was slower: 256 workgroups then hit the same few memory channels at once)
-  int qi = 0, sub = 0, sbuf = 0;  // 64-row step, tile inside it, set of per-row scalars in use
-  while (qi < n_qt && !visible(qi)) ++qi;
-  if (PF == 1 && qi < n_qt) fetch(qi * 64);
-  if (kDma && qi < n_qt) {
-    issue(qi * 64, 0);
-    small_fetch(qi * 64);
-    small_stash(0);
-  }
-  while (qi < n_qt) {
-    // what comes next: the other tile of this 64-row step, or the first tile of the next visible step
-    int nxi = qi, nsub = sub + 1;
-    if (nsub == NSUB) {
-      nsub = 0;
-      ++nxi;
-      while (nxi < n_qt && !visible(nxi)) ++nxi;
-    }
-    const int qt = qi, nxt = nxi;
-    const bool full = fully_visible(qt);
-    const bool have_next = nxi < n_qt;
-    if constexpr (kDma) {
-      // this wave's loads of the tile have landed; behind the barrier everybody's have, the per-row
-      // scalars written at the end of the last iteration are visible, and the other buffer is free
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (have_next) {
-        issue(nxt * 64 + nsub * QT, buf ^ 1);
-        if (nsub == 0) small_fetch(nxt * 64);
-      }
-      tile = sm8 + buf * SM::kBuf;
-      const int o = sbuf * (SM::kSmall / 4);
-      lse_s = const_cast<float*>(lse_s0) + o;
-      delta_s = lse_s + 64;
-      a1_s = reinterpret_cast<int*>(delta_s + 64);
-      b1_s = a1_s + 64; a2_s = b1_s + 64; b2_s = a2_s + 64;
-    } else {
-      __syncthreads();
-      if (PF) stash(); else direct(qt * 64);
-      __syncthreads();
-      if (PF && have_next) fetch(nxt * 64);
-    }
-    const int sub_now = sub;
-    qi = nxi;
-    sub = nsub;
-
-    // the two 32-row halves of the query tile one after the other (keeps 32 score
-    // registers live instead of 64)
-    // (head_dim 256 has no registers to spare for two unrolled halves in flight: a real loop there)
-#pragma unroll(kTR ? 1 : NQB)
-    for (int qbl = 0; qbl < NQB; ++qbl) {
-      const int qb = sub_now * NQB + qbl;  // 32-row half inside the 64-row step (per-row scalars); qbl: inside the LDS tile
-      // the scores start from -lse of their query row and dO V^T from -delta (LDS holds both
-      // negated): s - lse and dP - delta come out of the matrix pipe.  The Q tile is the scaled
-      // copy (bf16(q * scale * log2 e)), so the scores are base-2 exponents already
-      f32x16 st, dp;
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int q0 = qb * 32 + 8 * r4 + 4 * g;  // 4 consecutive query rows: one 16-byte LDS read each
-        const f32x4 ls = *reinterpret_cast<const f32x4*>(&lse_s[q0]);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) st[r4 * 4 + t] = ls[t];
-        if (kDoK) {
-          const f32x4 dl = *reinterpret_cast<const f32x4*>(&delta_s[q0]);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) dp[r4 * 4 + t] = dl[t];
-        } else {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) dp[r4 * 4 + t] = 0.f;
-        }
-      }
-      {
-        // Q (and, for dK, dO) row fragments through a ring of four registers: the read of
-        // fragment f + 4 follows the MFMA of fragment f, so no MFMA waits for LDS
-        constexpr int PER = kDoK ? 2 : 1;  // fragments per K step: Q [, dO]
-        constexpr int NF = PER * NKK;
-        constexpr int RG = SPX_DKV_RING;
-        bf16x8 fr[RG];
-        auto fread = [&](int f) {
-          if constexpr (kDma) {
-            const uint8_t* base = tile + ((PER == 2 && (f & 1)) ? SM::kOffdO : 0);
-            fr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                base + qbl * 32 * RBQ + (rdr ^ ((f / PER) * 32))));
-          } else {
-            const uint16_t* base = (PER == 2 && (f & 1)) ? dOs : Qs;
-            fr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                &base[(qb * 32 + col) * QS + g * 8 + (f / PER) * 16]));
-          }
-        };
-#pragma unroll
-        for (int f = 0; f < RG && f < NF; ++f) fread(f);
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          __builtin_amdgcn_sched_barrier(0);
-          if (PER == 2 && (f & 1)) dp = mfma32(fr[f % RG], vf[(f / PER) % NVF], dp);
-          else st = mfma32(fr[f % RG], kf[f / PER], st);
-          __builtin_amdgcn_sched_barrier(0);
-          if (f + RG < NF) fread(f + RG);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = fast_exp2(st[r]);
-      if (!full) {
-        // a real (scalar) branch: only tiles that straddle an interval edge pay for the mask
-        typedef __attribute__((ext_vector_type(4))) int i32x4;
-        pin_block(st);
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const int q0 = qb * 32 + 8 * r4 + 4 * g;
-          const i32x4 a1v = *reinterpret_cast<const i32x4*>(&a1_s[q0]);
-          const i32x4 b1v = *reinterpret_cast<const i32x4*>(&b1_s[q0]);
-          const i32x4 a2v = *reinterpret_cast<const i32x4*>(&a2_s[q0]);
-          const i32x4 b2v = *reinterpret_cast<const i32x4*>(&b2_s[q0]);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const bool ok = ((c >= a1v[t] && c < b1v[t]) || (c >= a2v[t] && c < b2v[t])) && (c < p.NKV);
-            if (!ok) st[r4 * 4 + t] = 0.f;
-          }
-        }
-        pin_block(st);
-      }
-      if (kDoK) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dp[r] *= st[r];
-      }
-      {
-        // dO^T / Q^T fragments through the same kind of ring; per (16-row step s2, D block db):
-        // dO^T [, Q^T]
-        constexpr int PER = (kDoV ? 1 : 0) + (kDoK ? 1 : 0);
-        constexpr int NF = PER * 2 * NDB;
-        constexpr int RG = SPX_DKV_RING;
-        bf16x8 fr[RG];
-        auto fread = [&](int f) {
-          const int e = f / PER, s2 = e / NDB, db = e % NDB;
-          const bool is_q = kDoK && (!kDoV || (f % PER) == 1);
-          if constexpr (kTR) {
-            const uint8_t* base = tile + (is_q ? 0 : SM::kOffdO) + (qbl * 32 + s2 * 16) * RBQ;
-            const i16x4 lo = lds_read_tr16(base + (rt0 ^ (db * 64)));
-            const i16x4 hi = lds_read_tr16(base + (rt1 ^ (db * 64)));
-            fr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-          } else if constexpr (kDma) {
-            const uint8_t* base = tile + (is_q ? SM::kOffQt : SM::kOffdOt);
-            fr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                base + db * 32 * RBT + (rdt ^ ((qbl * 2 + s2) * 32))));
-          } else {
-            const uint16_t* base = is_q ? Qts : dOts;
-            fr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                &base[(db * 32 + col) * TS + (qb * 2 + s2) * 16 + 8 * g]));
-          }
-        };
-#pragma unroll
-        for (int f = 0; f < RG && f < NF; ++f) fread(f);
-        bf16x8 pb = pack8(st, 0), sb8 = pack8(dp, 0);
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const int e = f / PER, s2 = e / NDB, db = e % NDB;
-          const bool is_q = kDoK && (!kDoV || (f % PER) == 1);
-          if (f == PER * NDB) { pb = pack8(st, 8); sb8 = pack8(dp, 8); }
-          __builtin_amdgcn_sched_barrier(0);
-          if (is_q) acc_dk[db % NAK] = mfma32(fr[f % RG], sb8, acc_dk[db % NAK]);
-          else acc_dv[db % NAV] = mfma32(fr[f % RG], pb, acc_dv[db % NAV]);
-          __builtin_amdgcn_sched_barrier(0);
-          if (f + RG < NF) fread(f + RG);
-          (void)s2;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    if constexpr (kDma) {
-      // the per-row scalars of the next 64-row step go into the other set: nobody reads it before the
-      // barrier
-      if (nsub == 0) {
-        if (have_next) {
-          lse_s = const_cast<float*>(lse_s0); delta_s = lse_s + 64;
-          a1_s = reinterpret_cast<int*>(delta_s + 64); b1_s = a1_s + 64; a2_s = b1_s + 64; b2_s = a2_s + 64;
-          small_stash(sbuf ^ 1);
-        }
-        sbuf ^= 1;
-      }
-      buf ^= 1;
-    }
-  }
-
-  if (c < p.NKV) {
-    float* krow = dKp + ((int64_t)h * p.NKV + c) * D + 4 * g;
-    float* vrow = dVp + ((int64_t)h * p.NKV + c) * D + 4 * g;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        if (kDoK) {
-          const f32x16& a = acc_dk[db % NAK];
-          f32x4 wk = {a[r4 * 4 + 0], a[r4 * 4 + 1], a[r4 * 4 + 2], a[r4 * 4 + 3]};
-          *reinterpret_cast<f32x4*>(krow + db * 32 + 8 * r4) = wk;
-        }
-        if (kDoV) {
-          const f32x16& a = acc_dv[db % NAV];
-          f32x4 wv = {a[r4 * 4 + 0], a[r4 * 4 + 1], a[r4 * 4 + 2], a[r4 * 4 + 3]};
-          *reinterpret_cast<f32x4*>(vrow + db * 32 + 8 * r4) = wv;
-        }
-      }
-  }
-}
-
-// ---------------------------------------------------------------- dK / dV, wave-specialised
-// The work of attn_bwd_dkv_kernel for head_dim <= 128 (both gradients in one pass), split over
-// TWO waves per SIMD that run different halves of it, so that each SIMD has a wave for the matrix
-// pipe while the other is in its vector phase, and every MFMA works on plain vector registers:
-//   producer wave i (waves 0-3): keeps K / V fragments of its 32 keys; per 32-row query tile
-//     S = Q' K^T - lse and dP = dO V^T - delta (16 MFMAs at head_dim 128), P = exp2(S), dS = P dP,
-//     both rounded to bf16 in the B-operand layout and handed over through a 4 KB LDS slot;
-//   consumer wave i (waves 4-7, same SIMD): keeps the dK / dV accumulators of those 32 keys
-//     (128 registers); per tile dV^T += dO^T P and dK^T += Q'^T dS (16 MFMAs) from the slot.
-// Both roles read the SAME row-major query tile (32 rows of Q' and of dO): the consumers take
-// their A operands (dO^T, Q'^T fragments) with transposing LDS reads (ds_read_b64_tr_b16), so no
-// transposed copy of the queries exists in memory.  Everything a step needs comes global -> LDS
-// directly, kAhead tiles ahead, into a ring of kStages buffers: the tile, and the per-row scalars
-// (-lse, -delta: the C operands of the score products; the mask interval ends).  In step b the
-// producers turn the scores of tile b (computed one step earlier) into P and dS first, while the
-// consumers' MFMAs of tile b - 1 run, and compute the scores of tile b + 1 after that.  One
-// workgroup barrier per step; slots are double buffered.
-template <int D>
-struct DkvWsSmem {
-  static constexpr int kStages = 6;
-  static constexpr int kAhead = 4;                     // tile b + kAhead is issued in step b
-  static constexpr int kTile = 2 * 32 * D * 2;         // Q', dO: 32 rows of D each
-  static constexpr int kSlot = 16 * 64 * 4;            // 16 registers of 64 lanes
-  static constexpr int kOffSlot = kStages * kTile;
-  static constexpr int kOffSmall = kOffSlot + 4 * 2 * kSlot;
-  static constexpr int kSmall = 6 * 32 * 4;            // -lse, -delta, a1, b1, a2, b2 of 32 rows
-  static constexpr int kSets = 8;                      // sets of per-row scalars (tile k: set k % 8)
-  static constexpr int kOffList = kOffSmall + kSets * kSmall + 256;  // (+ a spare area)
-  static constexpr int kListCap = 2048;                // visible 64-row tiles per key block, at most
-  static constexpr int kList = (kListCap + 1) * 4;     // ... their list, closed by an end mark
-  static constexpr int kBytes = kOffList + 2 * kList + 64;  // two key blocks; scratch of the list builder
-  static constexpr uint32_t kListEnd = 0x7fffffffu;
-  static_assert(kStages >= kAhead + 2, "a buffer is free two steps after its tile's scores");
-};
-
-// Values a non-inlined device function receives arrive in vector registers; these make them
-// wave-uniform (scalar registers) again, which addresses of the global -> LDS loads must be.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <typename T>
-__device__ __forceinline__ T* uni(T* q) {
-  const uint64_t a = reinterpret_cast<uint64_t>(q);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-  return reinterpret_cast<T*>(((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ int64_t uni(int64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-
-
-// One role of the kernel as a function of its own (not inlined): the register allocation of the
-// producers (K / V fragments, scores) and of the consumers (128 accumulator registers) then do not
-// add up.  Both roles walk the same sequence of steps and meet at the same barriers.
-template <int D, bool PRODUCER>
-__device__ __attribute__((noinline)) void dkv_ws_role(
-    const AttnParams& p_in, const uint16_t* dO_in, int NQp_in, const float* neg_in,
-    const int32_t* mrows_in, float* dKp_in, float* dVp_in) {
-  using SM = DkvWsSmem<D>;
-  extern __shared__ __attribute__((aligned(16))) uint8_t ws_smem[];
-  AttnParams p;
-  p.Q = uni(p_in.Q); p.q_hs = uni(p_in.q_hs);
-  p.K = uni(p_in.K); p.k_hs = uni(p_in.k_hs);
-  p.V = uni(p_in.V); p.v_hs = uni(p_in.v_hs);
-  p.a1 = nullptr; p.b1 = nullptr; p.a2 = nullptr; p.b2 = nullptr;
-  p.NQ = uni(p_in.NQ); p.T = uni(p_in.T); p.NKV = uni(p_in.NKV); p.NKVp = uni(p_in.NKVp);
-  p.n_extra = uni(p_in.n_extra); p.Hq = uni(p_in.Hq); p.Hkv = uni(p_in.Hkv);
-  p.scale_log2e = p_in.scale_log2e; p.scaling = p_in.scaling;
-  const uint16_t* __restrict__ dO = uni(dO_in);
-  const int NQp = uni(NQp_in);
-  const float* __restrict__ neg = uni(neg_in);        // -lse [Hq][NQp], -delta [Hq][NQp]
-  const int32_t* __restrict__ mrows = uni(mrows_in);  // interval ends of every row, [4][NQp]
-  float* __restrict__ dKp = uni(dKp_in);
-  float* __restrict__ dVp = uni(dVp_in);
-
-  constexpr bool producer = PRODUCER;
-  constexpr int NKK = D / 16, NDB = D / 32;
-  constexpr int KB = 128;                                 // keys per workgroup
-  constexpr int RBQ = D * 2, CKQ = RBQ / 16;              // bytes / 16-byte chunks per row of Q' and dO
-  constexpr int NLQ = 32 * RBQ / 1024;                    // 1 KB wave loads per 32-row operand
-  constexpr int LPW = 2 * NLQ / 4;                        // tile loads per consumer wave (they issue them all)
-  constexpr int kLoads = LPW + 1;                         // ... plus one of per-row scalars
-  constexpr int RG = 4;
-  constexpr int NS = SM::kStages, AH = SM::kAhead;
-  static_assert(LPW >= 1 && 2 * NLQ % 4 == 0, "every consumer wave issues the same number of loads per tile");
-  // A workgroup takes key blocks i and n_kb - 1 - i of one head, one after the other: under a causal
-  // mask block i is seen by all later query tiles and its partner by correspondingly few, so every
-  // workgroup walks about the same number of tiles.
-  const int n_kb = (p.NKV + KB - 1) / KB, n_pair = (n_kb + 1) / 2;
-  int h, pair;
-  if (SPX_DKV_XCD && p.Hq % 8 == 0) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    h = xcd + 8 * (slot / n_pair);
-    pair = slot % n_pair;
-  } else {
-    h = blockIdx.x % p.Hq;
-    pair = blockIdx.x / p.Hq;
-  }
-  const int kvh = h / (p.Hq / p.Hkv);
-  for (int part = 0; part < 2; ++part) {
-  const int kb_idx = part == 0 ? pair : n_kb - 1 - pair;
-  if (part == 1) {
-    if (kb_idx == pair) break;   // the middle block of an odd count has no partner
-    __syncthreads();             // everybody is done with the ring, the slots and the sets
-  }
-  const int n0 = kb_idx * KB;
-  const int key_last = min(n0 + KB - 1, p.NKV - 1);
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
-  const int pw = wave & 3;                 // pair index: the 32 keys of this wave
-  const int g = lane >> 5, col = lane & 31;
-  const int c = n0 + pw * 32 + col;
-  const int cc = c < p.NKV ? c : p.NKV - 1;
-  const int n_qt = (p.NQ + 63) / 64;
-
-  // the steps: the two 32-row halves of every 64-row query tile that sees the block, in order.  The
-  // kernel has listed those tiles in LDS (bit 31: every key of the block is visible to all rows of the
-  // tile); step k is half k & 1 of list entry k / 2.
-  const uint32_t* const lst = reinterpret_cast<const uint32_t*>(ws_smem + SM::kOffList + part * SM::kList);
-  const int s_end = n_qt * 2;
-  auto step_of = [&](uint32_t e, int k_) { return (e & 0x7fffffffu) == SM::kListEnd ? s_end : (int)(e & 0x7fffffffu) * 2 + (k_ & 1); };
-  const int n_vis = uni(reinterpret_cast<const int*>(ws_smem + SM::kOffList + 2 * SM::kList)[8 + part]);
-  auto entry = [&](int k_) { return lst[min(k_ >> 1, n_vis)]; };
-
-  // position of 16-byte chunk c of row r inside its LDS row: c ^ swz_r(r).  Row-wise 16-byte reads of 32
-  // rows (the producers) and the transposing reads of 4 + 4 rows x 64 bytes (the consumers) both
-  // spread evenly over the banks.
-  auto swz_r = [](int r) {
-    return CKQ == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3);
-  };
-  const uint32_t lds0 = (uint32_t)uni((int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ws_smem);
-  const u32x4 qres = make_rsrc(p.Q + (int64_t)h * p.q_hs, (uint32_t)((int64_t)p.NQ * RBQ));
-  const u32x4 dres = make_rsrc(dO + (int64_t)h * D, (uint32_t)((((int64_t)p.NQ - 1) * p.Hq * D + D) * 2));
-  // per-row scalars of a tile: -lse | -delta, a1 | b1, a2 | b2 (32 values each), one 256-byte load
-  // by each of consumer waves 0-2 (the fourth repeats the first into a spare area so that all count
-  // alike).  The consumers issue every load: they have time to spare, the producers do not.
-  const u32x4 nres = make_rsrc(neg + (int64_t)h * NQp, (uint32_t)((((int64_t)p.Hq + 1) * NQp) * 4));
-  const u32x4 mres = make_rsrc(mrows, (uint32_t)(4 * (int64_t)NQp * 4));
-  const bool sm_mask = pw == 1 || pw == 2;
-  const int sm_off = (lane & 31) * 4 + (lane >> 5) * (sm_mask ? NQp * 4 : p.Hq * NQp * 4) +
-                     (pw == 2 ? 2 * NQp * 4 : 0);
-  // this wave's loads of a tile: load li = pw + 4 j of the 2 * NLQ that make it (Q' first, then dO);
-  // rows past the last query read as zeros (and contribute nothing)
-  int ld_off[LPW], ld_mul[LPW], ld_dst[LPW];
-#pragma unroll
-  for (int j = 0; j < LPW; ++j) {
-    const int li = pw + 4 * j;
-    const bool is_do = li >= NLQ;
-    const int l = is_do ? li - NLQ : li;
-    const int r = l * (1024 / RBQ) + lane / CKQ;
-    const int cofs = ((lane % CKQ) ^ swz_r(r)) * 16;
-    ld_mul[j] = is_do ? p.Hq * RBQ : RBQ;          // bytes per query row in global memory
-    ld_off[j] = r * ld_mul[j] + cofs;
-    ld_dst[j] = (is_do ? 32 * RBQ : 0) + l * 1024;
-  }
-  auto issue = [&](int s_, int buf, int set) __attribute__((always_inline)) {
-    const int mq = s_ * 32;
-    const uint32_t rb = lds0 + buf * SM::kTile;
-#pragma unroll
-    for (int j = 0; j < LPW; ++j)
-      load_to_lds16<0>(pw + 4 * j >= NLQ ? dres : qres, rb + ld_dst[j], ld_off[j] + mq * ld_mul[j], 0);
-    const uint32_t sb = lds0 + SM::kOffSmall + (pw == 3 ? SM::kSets * SM::kSmall : set * SM::kSmall + pw * 256);
-    load_to_lds4(sm_mask ? mres : nres, sb, sm_off + mq * 4, 0);
-  };
-  float* const small0 = reinterpret_cast<float*>(ws_smem + SM::kOffSmall);
-
-  // ---- role state
-  bf16x8 kf[producer ? NKK : 1], vf[producer ? NKK : 1];
-  f32x16 acc_dk[producer ? 1 : NDB], acc_dv[producer ? 1 : NDB];
-  if constexpr (producer) {
-    const uint16_t* krow = p.K + (int64_t)kvh * p.k_hs + (int64_t)cc * D + g * 8;
-    const uint16_t* vrow = p.V + (int64_t)kvh * p.v_hs + (int64_t)cc * D + g * 8;
-#pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
-      kf[kk] = as_bf16x8(*reinterpret_cast<const u32x4*>(krow + kk * 16));
-      vf[kk] = as_bf16x8(*reinterpret_cast<const u32x4*>(vrow + kk * 16));
-    }
-  } else {
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) { acc_dk[db][r] = 0.f; acc_dv[db][r] = 0.f; }
-  }
-  // producers: row `col`, 16-byte chunk 2 kk + g of Q' / dO
-  const int rdr = col * RBQ + ((g ^ swz_r(col)) * 16);
-  // consumers: lane s of 16-lane group G points at row 4 (G >> 1) + (s >> 2) (+ 8 for the second read) of
-  // a 16-row k step, bytes 8 (s & 3) of the 64-byte block 32 db + 16 (G & 1).  (The k index of the
-  // P / dS operand: element j of the lanes with g = lane / 32 is query row 4 g + j for j < 4 and
-  // 8 + 4 g + j - 4 after that, the accumulator layout of the score product.)
-  const int tG = lane >> 4, ts = lane & 15;
-  const int trow = 4 * (tG >> 1) + (ts >> 2);
-  const int tcl = 2 * (tG & 1) + ((ts & 3) >> 1);
-  const int rt0 = trow * RBQ + ((tcl ^ swz_r(trow)) * 16) + (ts & 1) * 8;
-  const int rt1 = (trow + 8) * RBQ + ((tcl ^ swz_r(trow + 8)) * 16) + (ts & 1) * 8;
-  uint8_t* const slot0 = ws_smem + SM::kOffSlot + pw * 2 * SM::kSlot;
-
-  // ---- the producers' two halves of a tile (kIdx: its index in the sequence of steps)
-  f32x16 st, dp;      // scores / dP of the tile in work
-  f32x16 stn, dpn;    // -lse, -delta of the next tile (the C operands of its first products)
-  constexpr int NFP = 2 * NKK;
-  bf16x8 pfr[RG];
-  const uint8_t* ptile = ws_smem;
-  auto pfread = [&](int f) __attribute__((always_inline)) {
-    pfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-        ptile + ((f & 1) ? 32 * RBQ : 0) + (rdr ^ ((f / 2) * 32))));
-  };
-  // first half: the LDS reads whose results the products start from (issued before the soft-max half
-  // of the previous tile, so that they are back when it ends)
-  auto score_begin = [&](int buf, int set) __attribute__((always_inline)) {
-    ptile = ws_smem + buf * SM::kTile;
-    const float* const lse_s = small0 + set * (SM::kSmall / 4);
-    const float* const delta_s = lse_s + 32;
-#pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const int q0 = 8 * r4 + 4 * g;  // 4 consecutive query rows: one 16-byte LDS read each
-      const f32x4 ls = *reinterpret_cast<const f32x4*>(&lse_s[q0]);
-      const f32x4 dl = *reinterpret_cast<const f32x4*>(&delta_s[q0]);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) { stn[r4 * 4 + t] = ls[t]; dpn[r4 * 4 + t] = dl[t]; }
-    }
-#pragma unroll
-    for (int f = 0; f < RG; ++f) pfread(f);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto score_finish = [&]() __attribute__((always_inline)) {
-    SPX_DKV_PRIO_MFMA();
-#pragma unroll
-    for (int f = 0; f < NFP; ++f) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (f & 1) dp = mfma32(pfr[f % RG], vf[producer ? f / 2 : 0], f == 1 ? dpn : dp);
-      else st = mfma32(pfr[f % RG], kf[producer ? f / 2 : 0], f == 0 ? stn : st);
-      __builtin_amdgcn_sched_barrier(0);
-      if (f + RG < NFP) pfread(f + RG);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    SPX_DKV_PRIO_VALU();
-  };
-  auto soft_valu = [&](int set, int par, bool full) __attribute__((always_inline)) {
-    const int* const a1_s = reinterpret_cast<const int*>(small0 + set * (SM::kSmall / 4) + 64);
-    const int* const b1_s = a1_s + 32; const int* const a2_s = b1_s + 32; const int* const b2_s = a2_s + 32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) st[r] = fast_exp2(st[r]);
-    if (!full) {
-      typedef __attribute__((ext_vector_type(4))) int i32x4;
-      pin_block(st);
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int q0 = 8 * r4 + 4 * g;
-        const i32x4 a1v = *reinterpret_cast<const i32x4*>(&a1_s[q0]);
-        const i32x4 b1v = *reinterpret_cast<const i32x4*>(&b1_s[q0]);
-        const i32x4 a2v = *reinterpret_cast<const i32x4*>(&a2_s[q0]);
-        const i32x4 b2v = *reinterpret_cast<const i32x4*>(&b2_s[q0]);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const bool ok = ((c >= a1v[t] && c < b1v[t]) || (c >= a2v[t] && c < b2v[t])) && (c < p.NKV);
-          if (!ok) st[r4 * 4 + t] = 0.f;
-        }
-      }
-      pin_block(st);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dp[r] *= st[r];
-    // hand P and dS over: four 16-byte stores per lane, slot row = register quad, column = lane
-    uint8_t* const slot = slot0 + par * SM::kSlot + lane * 16;
-    *reinterpret_cast<bf16x8*>(slot + 0 * 1024) = pack8(st, 0);
-    *reinterpret_cast<bf16x8*>(slot + 1 * 1024) = pack8(st, 8);
-    *reinterpret_cast<bf16x8*>(slot + 2 * 1024) = pack8(dp, 0);
-    *reinterpret_cast<bf16x8*>(slot + 3 * 1024) = pack8(dp, 8);
-  };
-  // ---- the consumers' half: dV^T += dO^T P, dK^T += Q'^T dS
-  auto consume = [&](int buf, int par) __attribute__((always_inline)) {
-    const uint8_t* const tile = ws_smem + buf * SM::kTile;
-    const uint8_t* const slot = slot0 + par * SM::kSlot + lane * 16;
-    bf16x8 pb[2], sb[2];
-    pb[0] = *reinterpret_cast<const bf16x8*>(slot + 0 * 1024);
-    pb[1] = *reinterpret_cast<const bf16x8*>(slot + 1 * 1024);
-    sb[0] = *reinterpret_cast<const bf16x8*>(slot + 2 * 1024);
-    sb[1] = *reinterpret_cast<const bf16x8*>(slot + 3 * 1024);
-    SPX_DKV_PRIO_MFMA();
-    constexpr int NF = 2 * 2 * NDB;
-    i16x4 lo[RG], hi[RG];
-    // fragment f: even = dO^T (for dV), odd = Q'^T (for dK); e = f / 2: k step s2 = e / NDB, row block db
-    auto fread = [&](int f) {
-      const int e = f / 2, s2 = e / NDB, db = e % NDB;
-      const uint8_t* const base = tile + ((f & 1) ? 0 : 32 * RBQ) + s2 * 16 * RBQ;
-      lo[f % RG] = lds_read_tr16(base + (rt0 ^ (db * 64)));
-      hi[f % RG] = lds_read_tr16(base + (rt1 ^ (db * 64)));
-    };
-    auto frag = [&](int f) {
-      const i16x8 v = __builtin_shufflevector(lo[f % RG], hi[f % RG], 0, 1, 2, 3, 4, 5, 6, 7);
-      return __builtin_bit_cast(bf16x8, v);
-    };
-#pragma unroll
-    for (int f = 0; f < RG; ++f) fread(f);
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const int e = f / 2, s2 = e / NDB, db = e % NDB;
-      __builtin_amdgcn_sched_barrier(0);
-      if (f & 1) acc_dk[producer ? 0 : db] = mfma32(frag(f), sb[s2], acc_dk[producer ? 0 : db]);   // Q'^T dS
-      else acc_dv[producer ? 0 : db] = mfma32(frag(f), pb[s2], acc_dv[producer ? 0 : db]);         // dO^T P
-      __builtin_amdgcn_sched_barrier(0);
-      if (f + RG < NF) fread(f + RG);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    SPX_DKV_PRIO_VALU();
-  };
-
-  // ---- prologue.  Tile k of the sequence of steps lives in ring buffer k % kStages, its per-row
-  // scalars in set k % kSets, its P / dS in slot k % 2.
-  int sq[AH + 1];               // sq[i]: the step (tile) of sequence index b + i
-  bool fq[AH + 1];              // ... whether every key of the block is visible to all of its rows
-#pragma unroll
-  for (int i = 0; i <= AH; ++i) {
-    const uint32_t e = (uint32_t)uni((int)entry(i));
-    sq[i] = step_of(e, i);
-    fq[i] = (e >> 31) != 0;
-  }
-  uint32_t pref = entry(AH + 1);   // fetched one step before it joins the queue
-  int sC = s_end;               // the consumers' tile: b - 1
-  if constexpr (!producer) {
-#pragma unroll
-    for (int i = 0; i < AH; ++i)
-      if (sq[i] < s_end) issue(sq[i], i, i);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __syncthreads();
-  if constexpr (producer) {
-    if (sq[0] < s_end) { score_begin(0, 0); score_finish(); }
-  }
-  int rb = 0, kP = 0;           // ring buffer of tile b; b itself
-  auto wrap = [](int x) { return x >= NS ? x - NS : x; };
-  for (;; ++kP) {
-    const bool p_active = sq[0] < s_end, c_active = sC < s_end;
-    if (!p_active && !c_active) break;
-    // tile b + 1 has landed when at most the loads of tiles b + 2 .. b + kAhead - 1 are in flight
-    static_assert(AH == 4, "the wait below counts two tiles");
-    if constexpr (!producer) {
-      const int later = (sq[2] < s_end ? 1 : 0) + (sq[3] < s_end ? 1 : 0);
-      if (later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");
-      else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();
-    if constexpr (producer) {
-      if (p_active) {
-        if (sq[1] < s_end) score_begin(wrap(rb + 1), (kP + 1) & (SM::kSets - 1));
-        soft_valu(kP & (SM::kSets - 1), kP & 1, fq[0]);
-        if (sq[1] < s_end) score_finish();
-      }
-    } else {
-      if (c_active) {
-        consume(wrap(rb + NS - 1), (kP - 1) & 1);
-      }
-      // tile b + kAhead into the buffer tile b - 2 left behind
-      if (sq[AH] < s_end) issue(sq[AH], wrap(rb + AH), (kP + AH) & (SM::kSets - 1));
-    }
-    // next step
-    sC = sq[0];
-#pragma unroll
-    for (int i = 0; i < AH; ++i) { sq[i] = sq[i + 1]; fq[i] = fq[i + 1]; }
-    {
-      const uint32_t e = (uint32_t)uni((int)pref);
-      sq[AH] = step_of(e, kP + 1 + AH);
-      fq[AH] = (e >> 31) != 0;
-      pref = entry(kP + 2 + AH);
-    }
-    rb = wrap(rb + 1);
-  }
-
-  if constexpr (!producer) if (c < p.NKV) {
-    float* krow = dKp + ((int64_t)h * p.NKV + c) * D + 4 * g;
-    float* vrow = dVp + ((int64_t)h * p.NKV + c) * D + 4 * g;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const f32x4 wk = {acc_dk[db][r4 * 4 + 0], acc_dk[db][r4 * 4 + 1], acc_dk[db][r4 * 4 + 2], acc_dk[db][r4 * 4 + 3]};
-        const f32x4 wv = {acc_dv[db][r4 * 4 + 0], acc_dv[db][r4 * 4 + 1], acc_dv[db][r4 * 4 + 2], acc_dv[db][r4 * 4 + 3]};
-        *reinterpret_cast<f32x4*>(krow + db * 32 + 8 * r4) = wk;
-        *reinterpret_cast<f32x4*>(vrow + db * 32 + 8 * r4) = wv;
-      }
-  }
-  }  // part
-}
-
-template <int D>
-__global__ __launch_bounds__(512, 1) void attn_bwd_dkv_ws_kernel(
-    AttnParams p, const uint16_t* __restrict__ dO, int NQp, const float* __restrict__ neg,
-    const int32_t* __restrict__ mrows, const int32_t* __restrict__ tile_bounds,
-    float* __restrict__ dKp, float* __restrict__ dVp) {
-  using SM = DkvWsSmem<D>;
-  extern __shared__ __attribute__((aligned(16))) uint8_t ws_smem[];
-  // ---- the visible query tiles of both key blocks, in order, into LDS (all 512 threads)
-  {
-    constexpr int KB = 128;
-    const int n_kb = (p.NKV + KB - 1) / KB, n_pair = (n_kb + 1) / 2;
-    const int pair = (SPX_DKV_XCD && p.Hq % 8 == 0) ? (int)(blockIdx.x >> 3) % n_pair : (int)blockIdx.x / p.Hq;
-    const int n_qt = (p.NQ + 63) / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int* const wtot = reinterpret_cast<int*>(ws_smem + SM::kOffList + 2 * SM::kList);
-    for (int part = 0; part < 2; ++part) {
-      const int kb_idx = part == 0 ? pair : n_kb - 1 - pair;
-      const int n0 = kb_idx * KB, key_last = min(n0 + KB - 1, p.NKV - 1);
-      uint32_t* const lst = reinterpret_cast<uint32_t*>(ws_smem + SM::kOffList + part * SM::kList);
-      int base = 0;
-      for (int q0 = 0; q0 < n_qt; q0 += 512) {
-        const int qt = q0 + tid;
-        bool vis = false, full = false;
-        if (qt < n_qt) {
-          const int32_t* tb = tile_bounds + qt * 8;
-          vis = (tb[0] <= key_last && tb[3] > n0) || (tb[4] <= key_last && tb[7] > n0);
-          full = (tb[1] <= n0 && tb[2] >= n0 + KB) || (tb[5] <= n0 && tb[6] >= n0 + KB);
-        }
-        const unsigned long long m = __ballot(vis);
-        const int before = __popcll(m & ((1ull << lane) - 1));
-        if (lane == 0) wtot[wave] = __popcll(m);
-        __syncthreads();
-        int off = base, all = 0;
-        for (int w = 0; w < 8; ++w) {
-          if (w < wave) off += wtot[w];
-          all += wtot[w];
-        }
-        if (vis) lst[off + before] = (uint32_t)qt | (full ? 0x80000000u : 0u);
-        base += all;
-        __syncthreads();
-      }
-      if (tid == 0) {
-        lst[base] = SM::kListEnd;
-        wtot[8 + part] = base;
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 256)
-    dkv_ws_role<D, true>(p, dO, NQp, neg, mrows, dKp, dVp);
-  else
-    dkv_ws_role<D, false>(p, dO, NQp, neg, mrows, dKp, dVp);
-}
-
-// dK[kvh, c, :] = scaling * sum_{h in group} dKp[h, c, :],  dV likewise (no scaling); bf16 out.
-// `accumulate`: what dK / dV hold is added (in fp32, one rounding).
+// dK[kvh, c, :] = scaling * sum of the partial results of the head units of kvh (n_hu / Hkv of them in each of n_sum
+// sets), dV likewise (no scaling); bf16 out.  `accumulate`: what dK / dV hold is added (in fp32, one rounding).
 __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(
-    const float* __restrict__ dKp, const float* __restrict__ dVp, int NKV, int D, int Hq, int Hkv,
+    const float* __restrict__ dKp, const float* __restrict__ dVp, int NKV, int D, int n_hu, int n_sum, int Hkv,
     float scaling, uint16_t* __restrict__ dK, int64_t dk_hs, uint16_t* __restrict__ dV, int64_t dv_hs,
     int accumulate) {
   const int64_t per_head = (int64_t)NKV * D / 4;  // float4 items
@@ -2173,13 +1139,14 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(
   if (idx >= per_head * Hkv) return;
   const int kvh = (int)(idx / per_head);
   const int64_t off = (idx % per_head) * 4;
-  const int group = Hq / Hkv;
+  const int units = n_hu / Hkv;
   f32x4 sk = {0, 0, 0, 0}, sv = {0, 0, 0, 0};
-  for (int hh = 0; hh < group; ++hh) {
-    const int64_t base = ((int64_t)(kvh * group + hh) * NKV) * D + off;
-    sk += *reinterpret_cast<const f32x4*>(dKp + base);
-    sv += *reinterpret_cast<const f32x4*>(dVp + base);
-  }
+  for (int s = 0; s < n_sum; ++s)
+    for (int u = 0; u < units; ++u) {
+      const int64_t base = ((int64_t)(s * n_hu + kvh * units + u) * NKV) * D + off;
+      sk += *reinterpret_cast<const f32x4*>(dKp + base);
+      sv += *reinterpret_cast<const f32x4*>(dVp + base);
+    }
   sk *= scaling;
   u32x2 wk, wv;
   if (accumulate) {
@@ -2296,62 +1263,92 @@ __global__ __launch_bounds__(256) void ttt_attn_bwd_diag_kernel(
 // ---------------------------------------------------------------- launchers
 static int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
-#define SPX_FWD_CFG 1, 4, 2
-#define SPX_DQ_CFG 1, 4, 4
-// head_dim 256: the next tile is prefetched into registers as well; the few registers that
-// spill cost far less than exposing the global-load latency with one workgroup per CU
-#define SPX_FWD256_PF 2
-#define SPX_DQ256_PF 4
-#define SPX_DKV_CFG 4, 2
-// (sub-blocks per wave, waves per workgroup, register prefetch) of the forward / dQ kernels,
-// (waves per workgroup, register prefetch) of the dK/dV kernel
-constexpr int cfg_nsb(int nsb, int, int) { return nsb; }
-constexpr int cfg_nw(int, int nw, int) { return nw; }
-constexpr int cfg_pf(int, int, int pf) { return pf; }
-constexpr int cfg_nw(int nw, int) { return nw; }
-constexpr int cfg_pf(int, int pf) { return pf; }
-constexpr int kFwdNSB = cfg_nsb(SPX_FWD_CFG), kFwdNW = cfg_nw(SPX_FWD_CFG), kFwdPF = cfg_pf(SPX_FWD_CFG);
-constexpr int kDqNSB = cfg_nsb(SPX_DQ_CFG), kDqNW = cfg_nw(SPX_DQ_CFG), kDqPF = cfg_pf(SPX_DQ_CFG);
-constexpr int kDkvNW = cfg_nw(SPX_DKV_CFG), kDkvPF = cfg_pf(SPX_DKV_CFG);
+constexpr int kFwdNSB = 1, kFwdNW = 4, kDqNSB = 1, kDqNW = 4;  // 32-row sub-blocks per wave, waves per workgroup
 
-static int64_t fwd_workspace_bytes(int64_t NKV, int Hkv, int D) {
-  return round_up((int64_t)Hkv * D * round_up(NKV, 128) * 2, 256);
+// The split of the dK / dV work with the least estimated time, in steps of 32 query rows (0.8 us).  A workgroup's key
+// block costs its steps (on average half the rows of a causal mask, at most all of them) and 17 steps for its start and
+// its results.  Pairs of key blocks are equally long, so they run in rounds of `slots` workgroups; single blocks, the
+// long ones first, keep the slots busy up to a tail of 0.65 units, or take as long as the longest.  More heads per
+// workgroup: fewer starts, and fewer partial results to write and to sum (3.5 TB/s); but no fewer head units than XCDs, or
+// workgroups far apart in the sequence share an L2 (16384 rows, 16 heads of 256: 3900 us with one or two heads, 4570 with
+// eight).
+// Measured (us, kernel + sum): 8192 rows, 64 heads of 128: 2217 with one head and pairs, 1998 with eight heads; 4096, 32
+// heads of 128: 306 -> 281 with two heads; 3001: 222 -> 184 with two heads, single; 1024: 63 -> 50 single; 1024, 16 heads
+// of 256: 60 -> 48 single.  (Cutting the query rows of a block into parts on top of that never paid: the second set of
+// partial results costs more than the idle compute units.)
+static DkvPlan dkv_plan(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
+  const int KB = D == 64 ? DkvCfg<64>::KB : D == 128 ? DkvCfg<128>::KB : DkvCfg<256>::KB, cap = DkvCfg<128>::kListCap;
+  const int slots = 256 * (D == 64 ? 2 : 1), group = Hq / Hkv;
+  DkvPlan pl;
+  pl.n_kb = (int)((NKV + KB - 1) / KB);
+  pl.windows = (int)(((NQ + 63) / 64 + cap - 1) / cap);
+  pl.heads = 1;
+  pl.paired = 0;
+  const double avg = ((double)NQ / 32 + 4) / 2, start = 17;
+  double best = 1e30;
+  for (int h = 1; h <= group && pl.windows == 1; h *= 2) {
+    const int n_hu = Hq / h;
+    if (group % h || (h > 1 && n_hu % 8)) continue;
+    const double sum = (double)n_hu * (double)NKV * D * 8 / 3.5e6 / 0.8;
+    const double unit = h * avg + start;
+    const double single = std::max(pl.n_kb * n_hu <= slots ? 0. : pl.n_kb * n_hu * unit / slots + 0.65 * unit,
+                                   2 * h * avg + start + 12) + sum;
+    const double pairs = (double)(((pl.n_kb + 1) / 2 * n_hu + slots - 1) / slots) * 2 * (1.08 * h * avg + start) + sum;
+    if (single < best) { best = single; pl.heads = h; pl.paired = 0; }
+    if (pairs < best) { best = pairs; pl.heads = h; pl.paired = 1; }
+  }
+  pl.n_hu = Hq / pl.heads;
+  pl.n_k = pl.paired ? (pl.n_kb + 1) / 2 : pl.n_kb * pl.windows;
+  return pl;
+}
+
+// Forward calls of little work take V^T from transposing reads, larger ones from a copy: the copy pays above about 60 us of
+// products at head_dim <= 128 and 16 us at 256 (at 800 TFLOP/s of a causal mask).  Measured, copy + kernel against
+// transposing reads: 512 rows, 32 heads of 64 16.9 / 13.4 us, 2048 of 128 57.7 / 58.3, 4096 of 128 145 / 147, 16384 rows of
+// 16 heads of 256 2485 / 3072.
+static bool fwd_tr(int64_t NQ, int64_t NKV, int Hq, int D) {
+  return 2. * (double)Hq * (double)NQ * (double)NKV * D < (D > 128 ? 16. : 60.) * 8e8;
+}
+static int64_t fwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
+  return fwd_tr(NQ, NKV, Hq, D) ? 256 : round_up((int64_t)Hkv * D * round_up(NKV, 128) * 2, 256);
 }
 static int64_t bwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
-  const int64_t NKVp = round_up(NKV, 128), NQp = round_up(NQ, 128);
-  int64_t b = (int64_t)Hkv * D * NKVp * 2;          // K^T
-  b += 2 * (int64_t)Hq * D * NQp * 2;                // Q^T (scaled), dO^T
-  b = round_up(b, 256) + round_up((int64_t)Hq * NQ * 4, 256);       // delta
+  const int64_t NQp = round_up(NQ, 128);
+  int64_t b = round_up((int64_t)Hq * NQ * 4, 256);                  // delta
   b += round_up(((NQ + 63) / 64) * 32, 256);                        // tile bounds
-  b += 2 * round_up((int64_t)Hq * NKV * D * 4, 256);                // fp32 per-head dK, dV
+  b += 2 * round_up((int64_t)dkv_plan(NQ, NKV, Hq, Hkv, D).parts() * NKV * D * 4, 256);  // fp32 partial dK, dV
   b += round_up((int64_t)Hq * NQ * D * 2, 256);                     // Q scaled, row-major
   b += round_up(2 * (int64_t)Hq * NQp * 4, 256);                    // -lse, -delta in padded rows
   b += round_up(4 * NQp * 4, 256);                                  // interval ends of every row
   return b;
 }
 
-template <int D>
-static int launch_fwd(AttnParams p, void* workspace, uint16_t* O, float* lse, hipStream_t st,
-                      const char* fn) {
-  uint16_t* vt = reinterpret_cast<uint16_t*>(workspace);
-  dim3 tgrid((unsigned)(p.NKVp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hkv);
-  hipLaunchKernelGGL(transpose_bf16_kernel<false>, tgrid, dim3(64), 0, st, p.V, p.v_hs, (int64_t)D, p.NKV, D,
-                     vt, (int64_t)D * p.NKVp, (int64_t)p.NKVp, 1.f, nullptr);
+template <int D, bool TR>
+static int launch_fwd_as(AttnParams p, const uint16_t* vt, uint16_t* O, float* lse, hipStream_t st, const char* fn) {
   constexpr int BM = 32 * kFwdNSB * kFwdNW;
   const int n_qb = (p.NQ + BM - 1) / BM;
-  constexpr int PF = D > 128 ? (int)SPX_FWD256_PF : kFwdPF;
-  constexpr int smem = FwdSmem<D, kFwdNW, PF>::kBytes;
-  if (PF == 2 && ((int64_t)p.NKV * D * 2 >= (1ll << 31) || (int64_t)D * p.NKVp * 2 >= (1ll << 31))) {
+  constexpr int smem = FwdSmem<D, kFwdNW>::kBytes;
+  static std::atomic<uint64_t> lds_set;  // per instantiation, one bit per device
+  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>), smem, lds_set, fn))
+    return rc;
+  hipLaunchKernelGGL((attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kFwdNW), smem,
+                     st, p, vt, O, lse);
+  return check_launch(fn);
+}
+
+// workspace: room for V^T (fwd_workspace_bytes), or null: transposing reads whatever the size
+template <int D>
+static int launch_fwd(AttnParams p, void* workspace, uint16_t* O, float* lse, hipStream_t st, const char* fn) {
+  if ((int64_t)p.NKVp * D * 2 >= (1ll << 31)) {
     last_error() = std::string(fn) + ": keys of one head must span less than 2 GiB";
     return SPX_ERR_ARG;
   }
-  static std::atomic<uint64_t> lds_set;  // per head_dim instantiation, one bit per device
-  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, kFwdNW, PF>),
-                                  smem, lds_set, fn))
-    return rc;
-  hipLaunchKernelGGL((attn_fwd_kernel<D, kFwdNSB, kFwdNW, PF>), dim3((unsigned)(n_qb * p.Hq)),
-                     dim3(64 * kFwdNW), smem, st, p, vt, O, lse);
-  return check_launch(fn);
+  if (!workspace || fwd_tr(p.NQ, p.NKV, p.Hq, D)) return launch_fwd_as<D, true>(p, nullptr, O, lse, st, fn);
+  uint16_t* vt = reinterpret_cast<uint16_t*>(workspace);
+  dim3 tgrid((unsigned)(p.NKVp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hkv);
+  hipLaunchKernelGGL(transpose_bf16_kernel, tgrid, dim3(64), 0, st, p.V, p.v_hs, (int64_t)D, p.NKV, D,
+                     vt, (int64_t)D * p.NKVp, (int64_t)p.NKVp);
+  return launch_fwd_as<D, false>(p, vt, O, lse, st, fn);
 }
 
 template <int D>
@@ -2359,101 +1356,67 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
                       uint16_t* dQp, int64_t dq_hs, uint16_t* dKp, int64_t dk_hs, uint16_t* dVp,
                       int64_t dv_hs, void* workspace, hipStream_t st, const char* fn, int accumulate = 0) {
   const int NQp = (int)round_up(p.NQ, 128);
+  const DkvPlan pl = dkv_plan(p.NQ, p.NKV, p.Hq, p.Hkv, D);
   char* w = reinterpret_cast<char*>(workspace);
-  uint16_t* kt = reinterpret_cast<uint16_t*>(w);
-  // (the room behind K^T once held Q^T and dO^T; the layout of the workspace has not moved)
-  w += round_up(((int64_t)p.Hkv * D * p.NKVp + 2 * (int64_t)p.Hq * D * NQp) * 2, 256);
   float* delta = reinterpret_cast<float*>(w);
   w += round_up((int64_t)p.Hq * p.NQ * 4, 256);
   int32_t* tb = reinterpret_cast<int32_t*>(w);
   w += round_up(((p.NQ + 63) / 64) * 32, 256);
   float* dkp = reinterpret_cast<float*>(w);
-  w += round_up((int64_t)p.Hq * p.NKV * D * 4, 256);
+  w += round_up((int64_t)pl.parts() * p.NKV * D * 4, 256);
   float* dvp = reinterpret_cast<float*>(w);
-  w += round_up((int64_t)p.Hq * p.NKV * D * 4, 256);
+  w += round_up((int64_t)pl.parts() * p.NKV * D * 4, 256);
   uint16_t* qs = reinterpret_cast<uint16_t*>(w);  // bf16(q * scale * log2 e), [Hq][NQ][D]
   w += round_up((int64_t)p.Hq * p.NQ * D * 2, 256);
   float* neg = reinterpret_cast<float*>(w);       // -lse [Hq][NQp], -delta [Hq][NQp]
   w += round_up(2 * (int64_t)p.Hq * NQp * 4, 256);
   int32_t* mrows = reinterpret_cast<int32_t*>(w); // [4][NQp]
 
-  // (the dQ kernel's transposing-read mode takes its K^T fragments from the row-major K tile)
-  constexpr bool kNeedKt = (D > 128 ? (int)SPX_DQ256_PF : kDqPF) != 4;
-  dim3 tgrid((unsigned)(p.NKVp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hkv);
-  if (kNeedKt)
-    hipLaunchKernelGGL(transpose_bf16_kernel<false>, tgrid, dim3(64), 0, st, p.K, p.k_hs, (int64_t)D, p.NKV, D,
-                       kt, (int64_t)D * p.NKVp, (int64_t)p.NKVp, 1.f, nullptr);
-  dim3 qgrid((unsigned)(NQp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hq);
-  // (neither dK/dV kernel needs Q^T / dO^T: both transpose inside LDS.  The wave-specialised one lists the
-  // query tiles that see a key block in LDS, which bounds their number)
-  if (D <= 128 && (p.NQ + 63) / 64 > DkvWsSmem<(D <= 128 ? D : 128)>::kListCap) {
-    last_error() = std::string(fn) + ": more than " +
-                   std::to_string(64 * DkvWsSmem<(D <= 128 ? D : 128)>::kListCap) +
+  // (one list of query tiles in LDS; more rows than that are cut into windows at head_dim 256 only)
+  if (D <= 128 && (p.NQ + 63) / 64 > DkvCfg<D>::kListCap) {
+    last_error() = std::string(fn) + ": more than " + std::to_string(64 * DkvCfg<D>::kListCap) +
                    " query rows in one call at head_dim <= 128";
     return SPX_ERR_ARG;
   }
-  hipLaunchKernelGGL(transpose_bf16_kernel<true>, qgrid, dim3(64), 0, st, p.Q, p.q_hs, (int64_t)D, p.NQ, D,
-                     (uint16_t*)nullptr, (int64_t)D * NQp, (int64_t)NQp, p.scale_log2e, qs);
   // the dK/dV and diagonal-key kernels read the scaled queries: their scores are q' . k with no
   // factor of their own, and what they accumulate against q' carries scale * log2(e) once too
   // often: dK = ln 2 * sum dS q'
   AttnParams ps = p;
   ps.Q = qs;
   ps.q_hs = (int64_t)p.NQ * D;
-  if (NQp != p.NQ)  // the padding of the negated rows reads as zero
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((2 * (int64_t)p.Hq * NQp + 255) / 256)), dim3(256), 0,
-                       st, neg, 2 * (int64_t)p.Hq * NQp);
-  hipLaunchKernelGGL(attn_delta_kernel<D>, dim3((unsigned)(((int64_t)p.NQ * p.Hq + 15) / 16)), dim3(256),
-                     0, st, Op, dOp, p.NQ, p.Hq, delta, lse, NQp, neg);
-  hipLaunchKernelGGL(attn_tile_bounds_kernel, dim3((unsigned)(NQp / 64)), dim3(64), 0, st, p, tb, NQp, mrows);
+  const int row_blocks = (int)(((int64_t)p.Hq * NQp + 15) / 16);
+  hipLaunchKernelGGL(attn_bwd_prep_kernel<D>, dim3((unsigned)(row_blocks + (NQp / 64 + 3) / 4)), dim3(256), 0, st, p, Op,
+                     dOp, lse, NQp, row_blocks, qs, delta, neg, tb, mrows);
 
   constexpr int BM = 32 * kDqNSB * kDqNW;
   const int n_qb = (p.NQ + BM - 1) / BM;
   {
-    constexpr int kDqPFd = D > 128 ? (int)SPX_DQ256_PF : kDqPF;
-    constexpr int dq_smem = DqSmem<D, kDqNW, kDqPFd>::kBytes;
-    if (kDqPFd >= 3 && ((int64_t)p.NKV * D * 2 >= (1ll << 31) || (int64_t)D * p.NKVp * 2 >= (1ll << 31))) {
+    constexpr int dq_smem = DqSmem<D, kDqNW>::kBytes;
+    if ((int64_t)p.NKVp * D * 2 >= (1ll << 31)) {
       last_error() = std::string(fn) + ": keys of one head must span less than 2 GiB";
       return SPX_ERR_ARG;
     }
     static std::atomic<uint64_t> dq_lds_set;  // per head_dim instantiation, one bit per device
-    if (int rc = ensure_dynamic_lds(
-            reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, kDqNSB, kDqNW, kDqPFd>), dq_smem,
-            dq_lds_set, fn))
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, kDqNSB, kDqNW>), dq_smem,
+                                    dq_lds_set, fn))
       return rc;
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, kDqNSB, kDqNW, kDqPFd>), dim3((unsigned)(n_qb * p.Hq)),
-                       dim3(64 * kDqNW), dq_smem, st, p, dOp, kt, lse, delta, dQp, dq_hs);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, kDqNSB, kDqNW>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kDqNW), dq_smem,
+                       st, p, dOp, lse, delta, dQp, dq_hs);
   }
 
-  if (D > 128 && (int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31)) {
+  if ((int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31)) {
     last_error() = std::string(fn) + ": queries must span less than 2 GiB";
     return SPX_ERR_ARG;
   }
   static std::atomic<uint64_t> dkv_lds_set;  // per head_dim instantiation, one bit per device
-  if constexpr (D <= 128) {
-    // producer / consumer waves, two per SIMD (see attn_bwd_dkv_ws_kernel)
-    constexpr int smem = DkvWsSmem<D>::kBytes;
-    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dkv_ws_kernel<D>), smem,
-                                    dkv_lds_set, fn))
-      return rc;
-    const int n_pair_ws = ((p.NKV + 127) / 128 + 1) / 2;  // a workgroup takes two key blocks
-    hipLaunchKernelGGL((attn_bwd_dkv_ws_kernel<D>), dim3((unsigned)(n_pair_ws * p.Hq)), dim3(512), smem, st, ps,
-                       dOp, NQp, neg, mrows, tb, dkp, dvp);
-  } else {
-    // dK and dV in one pass over 64-row tiles of Q and dO alone (two buffers of two 32 KB tiles); the
-    // transposed operands come out of them through transposing LDS reads
-    const int n_kb = (p.NKV + 32 * kDkvNW - 1) / (32 * kDkvNW);
-    const dim3 kgrid((unsigned)(n_kb * p.Hq)), kblock(64 * kDkvNW);
-    constexpr size_t smem = DkvSmem<D, 0, 64, true>::kBytesDma;
-    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<D, kDkvNW, 4, 0>),
-                                    (int)smem, dkv_lds_set, fn))
-      return rc;
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<D, kDkvNW, 4, 0>), kgrid, kblock, smem, st, ps, dOp,
-                       (const uint16_t*)nullptr, (const uint16_t*)nullptr, NQp, lse, delta, tb, dkp, dvp);
-  }
+  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<D>), DkvCfg<D>::kBytes,
+                                  dkv_lds_set, fn))
+    return rc;
+  hipLaunchKernelGGL((attn_bwd_dkv_kernel<D>), dim3((unsigned)(pl.n_k * pl.n_hu)), dim3(512), DkvCfg<D>::kBytes, st,
+                     ps, dOp, NQp, neg, mrows, tb, pl, dkp, dvp);
   const int64_t items = (int64_t)p.NKV * D / 4 * p.Hkv;
   hipLaunchKernelGGL(attn_dkv_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, dkp,
-                     dvp, p.NKV, D, p.Hq, p.Hkv, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate);
+                     dvp, p.NKV, D, pl.n_hu, pl.windows, p.Hkv, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate);
   if (p.n_extra > 0) {
     const dim3 dgrid((unsigned)(((int64_t)p.T * p.Hkv + 15) / 16));
     // eight heads per K/V head in registers where they fit (head_dim <= 128), else four
@@ -2504,7 +1467,7 @@ extern "C" int spx_ttt_row_lo(const void* document_ids, int doc_kind, int64_t T,
 
 extern "C" int64_t spx_ttt_attn_workspace_bytes(int64_t T, int32_t Hq, int32_t Hkv, int32_t D,
                                                 int32_t backward) {
-  return backward ? bwd_workspace_bytes(T, T, Hq, Hkv, D) : fwd_workspace_bytes(T, Hkv, D);
+  return backward ? bwd_workspace_bytes(T, T, Hq, Hkv, D) : fwd_workspace_bytes(T, T, Hq, Hkv, D);
 }
 
 static AttnParams ttt_params(const void* q, int64_t q_hs, const void* k, int64_t k_hs, const void* v,
@@ -2521,28 +1484,37 @@ static AttnParams ttt_params(const void* q, int64_t q_hs, const void* k, int64_t
   return p;
 }
 
+// workspace: null = none (spx_ttt_attn_fwd_static)
+static int ttt_attn_fwd_impl(const char* fname, const void* q, int64_t q_head_stride, const void* k,
+                             int64_t k_head_stride, const void* v, int64_t v_head_stride, const int32_t* row_lo,
+                             int64_t T, int32_t ttt_step, int32_t Hq, int32_t Hkv, int32_t D, float scaling, void* out,
+                             float* lse, void* workspace, void* stream) {
+  if (!(ttt_step >= 0 && ttt_step < 64)) return fail_arg(fname, "0 <= ttt_step < 64");
+  if (!(q && k && v && row_lo && out && lse)) return fail_arg(fname, "null buffer");
+  if (q_head_stride < T * D) return fail_arg(fname, "q head stride smaller than T*D");
+  if (k_head_stride < (int64_t)(ttt_step + 1) * T * D || v_head_stride < (int64_t)(ttt_step + 1) * T * D)
+    return fail_arg(fname, "k/v head stride smaller than (ttt_step+1)*T*D");
+  if (q_head_stride % 8 || k_head_stride % 8 || v_head_stride % 8)
+    return fail_arg(fname, "head strides must be multiples of 8 elements");
+  if (!all_aligned16({q, k, v, out, workspace})) return fail_arg(fname, "buffers must be 16-byte aligned");
+  AttnParams p = ttt_params(q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step,
+                            Hq, Hkv, scaling);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (D == 256) return launch_fwd<256>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, fname);
+  if (D == 128) return launch_fwd<128>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, fname);
+  return launch_fwd<64>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, fname);
+}
+
 extern "C" int spx_ttt_attn_fwd(const void* q, int64_t q_head_stride, const void* k,
                                 int64_t k_head_stride, const void* v, int64_t v_head_stride,
                                 const int32_t* row_lo, int64_t T, int32_t ttt_step, int32_t Hq,
                                 int32_t Hkv, int32_t D, float scaling, void* out, float* lse,
                                 void* workspace, int64_t workspace_bytes, void* stream) {
   if (int rc = shape_checks(__func__, T, T, Hq, Hkv, D)) return rc;
-  SPX_REQUIRE(ttt_step >= 0 && ttt_step < 64, "0 <= ttt_step < 64");
-  SPX_REQUIRE(q && k && v && row_lo && out && lse && workspace, "null buffer");
-  SPX_REQUIRE(q_head_stride >= T * D, "q head stride smaller than T*D");
-  SPX_REQUIRE(k_head_stride >= (int64_t)(ttt_step + 1) * T * D &&
-              v_head_stride >= (int64_t)(ttt_step + 1) * T * D,
-              "k/v head stride smaller than (ttt_step+1)*T*D");
-  SPX_REQUIRE(q_head_stride % 8 == 0 && k_head_stride % 8 == 0 && v_head_stride % 8 == 0,
-              "head strides must be multiples of 8 elements");
-  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(T, Hkv, D), "workspace too small");
-  SPX_REQUIRE(all_aligned16({q, k, v, out, workspace}), "buffers must be 16-byte aligned");
-  AttnParams p = ttt_params(q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step,
-                            Hq, Hkv, scaling);
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (D == 256) return launch_fwd<256>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, __func__);
-  if (D == 128) return launch_fwd<128>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, __func__);
-  return launch_fwd<64>(p, workspace, reinterpret_cast<uint16_t*>(out), lse, st, __func__);
+  SPX_REQUIRE(workspace, "null buffer");
+  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(T, T, Hq, Hkv, D), "workspace too small");
+  return ttt_attn_fwd_impl(__func__, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq,
+                           Hkv, D, scaling, out, lse, workspace, stream);
 }
 
 #define SPX_REQ_FN(cond, what) do { if (!(cond)) return spx::fail_arg(fname, what); } while (0)
@@ -2630,7 +1602,7 @@ extern "C" int spx_span_attn_fwd(const void* q, int64_t q_head_stride, const voi
               "head stride smaller than T*D");
   SPX_REQUIRE(q_head_stride % 8 == 0 && k_head_stride % 8 == 0 && v_head_stride % 8 == 0,
               "head strides must be multiples of 8 elements");
-  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(T, Hkv, D), "workspace too small");
+  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(T, T, Hq, Hkv, D), "workspace too small");
   SPX_REQUIRE(all_aligned16({q, k, v, out, workspace}), "buffers must be 16-byte aligned");
   AttnParams p = span_params(q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, row_hi, T, Hq,
                              Hkv, scaling);
@@ -2677,36 +1649,9 @@ extern "C" int spx_span_attn_bwd(const void* q, int64_t q_head_stride, const voi
 }
 
 // ---------------------------------------------------------------- allocation-free variant
-// The forward's only scratch is the key-contiguous copy V^T [Hkv, D, round_up(T, 128)].  Here it
-// lives in a file-scope device array instead of a caller-owned workspace.  Every GPU holds its
-// own copy of the array at its own address: the address is looked up once per device with that
-// device current and kept; host code never uses the array's name as a pointer.
+// The forward as callers without an allocator use it.  It keeps nothing in memory; the limit is part of the entry
+// point's contract.
 constexpr int64_t kStaticScratchBytes = 16ll << 20;
-static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
-
-constexpr int kMaxDevices = 64;
-static std::atomic<void*> g_scratch_ptr[kMaxDevices];
-
-static int static_scratch(void** out, const char* fn) {
-  int dev = -1;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) {
-    last_error() = std::string(fn) + ": hipGetDevice: " + hipGetErrorString(e);
-    return SPX_ERR_HIP;
-  }
-  if (dev < 0 || dev >= kMaxDevices) return fail_arg(fn, "device ordinal out of range");
-  void* ptr = g_scratch_ptr[dev].load(std::memory_order_acquire);
-  if (!ptr) {
-    e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !ptr) {
-      last_error() = std::string(fn) + ": hipGetSymbolAddress: " + hipGetErrorString(e);
-      return SPX_ERR_HIP;
-    }
-    g_scratch_ptr[dev].store(ptr, std::memory_order_release);  // same value from every thread
-  }
-  *out = ptr;
-  return SPX_OK;
-}
 
 extern "C" int64_t spx_ttt_attn_fwd_static_max_bytes(void) { return kStaticScratchBytes; }
 
@@ -2716,15 +1661,11 @@ extern "C" int spx_ttt_attn_fwd_static(const void* q, int64_t q_head_stride, con
                                        int32_t Hq, int32_t Hkv, int32_t D, float scaling, void* out,
                                        float* lse, void* stream) {
   if (int rc = shape_checks(__func__, T, T, Hq, Hkv, D)) return rc;
-  if (fwd_workspace_bytes(T, Hkv, D) > kStaticScratchBytes)
-    return fail_arg(__func__, "Hkv * D * round_up(T, 128) * 2 bytes exceed the 16 MiB static scratch; "
+  if ((int64_t)Hkv * D * round_up(T, 128) * 2 > kStaticScratchBytes)
+    return fail_arg(__func__, "Hkv * D * round_up(T, 128) * 2 bytes exceed 16 MiB, the limit of this entry point; "
                               "use spx_ttt_attn_fwd with a caller-owned workspace");
-  void* ws = nullptr;
-  if (int rc = static_scratch(&ws, __func__)) return rc;
-  // every byte of V^T the kernel reads is rewritten by this call's transpose (padding columns
-  // included), so nothing of an earlier call has to be cleared
-  return spx_ttt_attn_fwd(q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq,
-                          Hkv, D, scaling, out, lse, ws, kStaticScratchBytes, stream);
+  return ttt_attn_fwd_impl(__func__, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq,
+                           Hkv, D, scaling, out, lse, nullptr, stream);
 }
 
 // ================================================================ DFlash entry points
@@ -2759,7 +1700,7 @@ extern "C" int spx_dflash_row_ranges(const void* document_ids, int doc_kind, int
 
 extern "C" int64_t spx_dflash_attn_workspace_bytes(int64_t T, int64_t NQ, int32_t Hq, int32_t Hkv,
                                                    int32_t D, int32_t backward) {
-  return backward ? bwd_workspace_bytes(NQ, T + NQ, Hq, Hkv, D) : fwd_workspace_bytes(T + NQ, Hkv, D);
+  return backward ? bwd_workspace_bytes(NQ, T + NQ, Hq, Hkv, D) : fwd_workspace_bytes(NQ, T + NQ, Hq, Hkv, D);
 }
 
 static AttnParams dflash_params(const void* q, int64_t q_hs, const void* k, int64_t k_hs, const void* v,
@@ -2791,7 +1732,7 @@ extern "C" int spx_dflash_attn_fwd(const void* q, int64_t q_head_stride, const v
               "k/v head stride smaller than (T+NQ)*D");
   SPX_REQUIRE(q_head_stride % 8 == 0 && k_head_stride % 8 == 0 && v_head_stride % 8 == 0,
               "head strides must be multiples of 8 elements");
-  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(T + NQ, Hkv, D), "workspace too small");
+  SPX_REQUIRE(workspace_bytes >= fwd_workspace_bytes(NQ, T + NQ, Hq, Hkv, D), "workspace too small");
   SPX_REQUIRE(all_aligned16({q, k, v, out, workspace}), "buffers must be 16-byte aligned");
   AttnParams p = dflash_params(q, q_head_stride, k, k_head_stride, v, v_head_stride, ctx_lo, ctx_hi,
                                blk_lo, blk_hi, T, NQ, Hq, Hkv, scaling);

@@ -439,3 +439,46 @@ def test_full_size_head_dim_256_sampled_rows():
     _check_sampled_rows(q, k, v, out, go, rows, heads,
                         lambda i: (kv_idx <= i) & (seq == seq[i]), d ** -0.5)
     _check_dv_checksum(v, go, hq)
+
+
+@pytest.mark.parametrize("t,hq,hkv,d,doc_len", [
+    (2112, 64, 8, 64, 2112),     # several query heads per workgroup of the dK/dV kernel
+    (1984, 64, 8, 128, 1984),    # ... in pairs of key blocks
+    (1999, 32, 8, 128, 1999),    # a ragged last key block with a partner
+    (1027, 24, 2, 128, 79),      # a group of twelve heads; documents shorter than a key block
+    (2085, 16, 2, 256, 2085),    # head_dim 256, one head per workgroup, forward out of a transposed copy of V
+    (4160, 16, 2, 256, 4160),    # ... two heads
+    (131136, 1, 1, 256, 64),     # more query tiles than one list holds: two windows
+])
+def test_large_splits_match_fp32(t, hq, hkv, d, doc_len):
+    """Sizes at which the backward cuts its work differently (heads per workgroup, pairs, windows) and the
+    forward reads V transposed or as it lies: output and gradients against fp32 attention, document by document."""
+    from speculators_amd.attention import create_ttt_mask, ttt_attention
+
+    g = torch.Generator(device="cuda").manual_seed(t)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q, k, v = (r(1, h, t, d).requires_grad_(True) for h in (hq, hkv, hkv))
+    go = r(1, t, hq, d)
+    doc = torch.arange(t, device="cuda") // doc_len
+    out = ttt_attention(q, k, v, create_ttt_mask(doc, t), d ** -0.5)
+    dq, dk, dv = torch.autograd.grad(out, (q, k, v), go)
+    ro, rq = torch.zeros(t, hq, d, device="cuda"), torch.zeros(hq, t, d, device="cuda")
+    rk, rv = torch.zeros(hkv, t, d, device="cuda"), torch.zeros(hkv, t, d, device="cuda")
+    whole = t // doc_len * doc_len
+    for lo, hi, n in ((0, whole, t // doc_len), (whole, t, 1)):
+        if hi == lo:
+            continue
+        m = (hi - lo) // n
+        hide = torch.ones(m, m, device="cuda", dtype=torch.bool).triu(1)
+        for h in range(hq):
+            kv = h * hkv // hq
+            x, y, z = (a[0, i, lo:hi].float().view(n, m, d).requires_grad_(True) for a, i in ((q, h), (k, kv), (v, kv)))
+            p = (x @ y.transpose(1, 2) * d ** -0.5).masked_fill(hide, -torch.inf).softmax(-1)
+            o = p @ z
+            gx, gy, gz = torch.autograd.grad(o, (x, y, z), go[0, lo:hi, h].float().view(n, m, d))
+            ro[lo:hi, h], rq[h, lo:hi] = o.detach().view(-1, d), gx.view(-1, d)
+            rk[kv, lo:hi] += gy.reshape(-1, d)
+            rv[kv, lo:hi] += gz.reshape(-1, d)
+    for name, got, want in (("out", out[0], ro), ("dq", dq[0], rq), ("dk", dk[0], rk), ("dv", dv[0], rv)):
+        err = ((got.detach().float() - want).norm() / want.norm()).item()
+        assert err < 1e-2, (name, err)
