@@ -168,39 +168,15 @@ def native():
     floats, None and HIP tensors (where C takes a pointer) and raises ``SpxError`` on a failed status."""
     global _native
     if _native is None:
-        load()
-        if os.environ.get("SPX_LIB_PATH"):
-            _native = _CtypesCalls(_lib)  # another build of the library than the one beside this file
-        else:
-            try:
-                from . import _spx_native as mod
-            except ImportError as exc:
-                raise SpxError("speculators_amd/_spx_native.so is missing: build it with "
-                               "`make -C speculators_amd/csrc`; there is no fallback path") from exc
-            mod.set_error(SpxError)
-            _native = mod
+        load()  # (first: the module then binds to this build of the library, whatever its path)
+        try:
+            from . import _spx_native as mod
+        except ImportError as exc:
+            raise SpxError("speculators_amd/_spx_native.so is missing: build it with "
+                           "`make -C speculators_amd/csrc`; there is no fallback path") from exc
+        mod.set_error(SpxError)
+        _native = mod
     return _native
-
-
-class _CtypesCalls:
-    """The functions of the binding module over a ``ctypes`` library."""
-
-    def __init__(self, lib):
-        self._lib = lib
-
-    def __getattr__(self, name):
-        fn = getattr(self._lib, name)
-        status = name not in RESTYPES and name not in ("spx_version", "spx_gemm_auto_tile")
-
-        def call_(*args):
-            rc = fn(*(ptr(a) if isinstance(a, torch.Tensor) else a for a in args))
-            if not status:
-                return rc
-            if rc != 0:
-                raise SpxError(f"{name} failed ({rc}): {self._lib.spx_last_error().decode()}")
-
-        setattr(self, name, call_)
-        return call_
 
 
 def call(name: str, *args) -> None:

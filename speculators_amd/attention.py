@@ -76,41 +76,9 @@ def _check_qkv(q, k, v, mask: TTTMask):
     return hq, hkv, t, d
 
 
-class _TTTAttention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, mask: TTTMask, scaling: float):
-        hq, hkv, t, d = _check_qkv(q, k, v, mask)
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        dev = q.device
-        out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
-        lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_fwd", q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), mask.row_lo, t, mask.ttt_step, hq, hkv, d,
-                  float(scaling), out, lse, ws, ws.numel(),
-                  _lib.stream_ptr(dev))
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.mask, ctx.scaling = mask, float(scaling)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse = ctx.saved_tensors
-        mask = ctx.mask
-        _, hq, t, d = q.shape
-        hkv = k.shape[1]
-        dev = q.device
-        dout = dout.to(torch.bfloat16).contiguous()
-        dq = torch.empty_like(q)
-        dk = torch.empty_like(k)
-        dv = torch.empty_like(v)
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call("spx_ttt_attn_bwd", q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), out, dout, lse,
-                  mask.row_lo, t, mask.ttt_step, hq, hkv, d, ctx.scaling,
-                  dq, dq.stride(1), dk, dk.stride(1), dv,
-                  dv.stride(1), ws, ws.numel(), _lib.stream_ptr(dev))
-        return dq, dk, dv, None, None
+def _ttt(q, k, v, mask: TTTMask, scaling: float):
+    _check_qkv(q, k, v, mask)
+    return _lib.native().attention(q, k, v, mask.row_lo, None, None, None, mask.total_seq_len, mask.ttt_step, scaling)
 
 
 class TTTKVCache:
@@ -289,7 +257,7 @@ def _at_kernel_head_dim(fn, q, k, v, mask, scaling):
 
 def ttt_attention(q, k, v, mask: TTTMask, scaling: float | None = None) -> torch.Tensor:
     """``[1, Hq, T, D]`` x ``[1, Hkv, (step+1)*T, D]`` -> ``[1, T, Hq, D]`` (bf16)."""
-    return _at_kernel_head_dim(_TTTAttention.apply, q, k, v, mask, scaling)
+    return _at_kernel_head_dim(_ttt, q, k, v, mask, scaling)
 
 
 @dataclass
@@ -332,51 +300,21 @@ def create_padding_span_mask(attention_mask: torch.Tensor) -> SpanMask:
                     b * n)
 
 
-class _SpanAttention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, mask: SpanMask, scaling: float):
-        if q.dim() != 4 or q.shape[0] != 1:
-            raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, T, D]")
-        if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
-            raise _lib.SpxError("the HIP attention kernels take bf16 q/k/v")
-        _, hq, t, d = q.shape
-        hkv = k.shape[1]
-        if t != mask.total_seq_len or k.shape[2] != t or v.shape != k.shape:
-            raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match a span mask over "
-                             f"{mask.total_seq_len} positions")
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        dev = q.device
-        out = torch.empty(1, t, hq, d, device=dev, dtype=torch.bfloat16)
-        lse = torch.empty(hq, t, device=dev, dtype=torch.float32)
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, False), device=dev, dtype=torch.uint8)
-        _lib.call("spx_span_attn_fwd", q, q.stride(1), k, k.stride(1), v,
-                  v.stride(1), mask.row_lo, mask.row_hi, t, hq, hkv, d, float(scaling),
-                  out, lse, ws, ws.numel(), _lib.stream_ptr(dev))
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.mask, ctx.scaling = mask, float(scaling)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse = ctx.saved_tensors
-        mask = ctx.mask
-        _, hq, t, d = q.shape
-        hkv = k.shape[1]
-        dev = q.device
-        dout = dout.to(torch.bfloat16).contiguous()
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = torch.empty(_workspace_bytes(t, hq, hkv, d, True), device=dev, dtype=torch.uint8)
-        _lib.call("spx_span_attn_bwd", q, q.stride(1), k, k.stride(1), v,
-                  v.stride(1), out, dout, lse, mask.row_lo,
-                  mask.row_hi, t, hq, hkv, d, ctx.scaling, dq, dq.stride(1),
-                  dk, dk.stride(1), dv, dv.stride(1), ws, ws.numel(),
-                  _lib.stream_ptr(dev))
-        return dq, dk, dv, None, None
+def _span(q, k, v, mask: SpanMask, scaling: float):
+    if q.dim() != 4 or q.shape[0] != 1:
+        raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, T, D]")
+    if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
+        raise _lib.SpxError("the HIP attention kernels take bf16 q/k/v")
+    t = q.shape[2]
+    if t != mask.total_seq_len or k.shape[2] != t or v.shape != k.shape:
+        raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match a span mask over "
+                         f"{mask.total_seq_len} positions")
+    return _lib.native().attention(q, k, v, mask.row_lo, mask.row_hi, None, None, t, 0, scaling)
 
 
 def span_attention(q, k, v, mask: SpanMask, scaling: float | None = None) -> torch.Tensor:
     """``[1, Hq, T, D]`` x ``[1, Hkv, T, D]`` -> ``[1, T, Hq, D]`` (bf16) under a ``SpanMask``."""
-    return _at_kernel_head_dim(_SpanAttention.apply, q, k, v, mask, scaling)
+    return _at_kernel_head_dim(_span, q, k, v, mask, scaling)
 
 
 def ttt_hip_attention_forward(module, query, key, value, attention_mask, scaling=None, **_kwargs):
@@ -440,57 +378,21 @@ def create_dflash_mask(document_ids: torch.Tensor, total_seq_len: int,
     return DFlashMask(bounds[0], bounds[1], bounds[2], bounds[3], total_seq_len, n_q)
 
 
-class _DFlashAttention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, mask: DFlashMask, scaling: float):
-        if q.dim() != 4 or q.shape[0] != 1:
-            raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, NQ, D]")
-        if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
-            raise _lib.SpxError("the HIP attention kernels take bf16 q/k/v")
-        _, hq, nq, d = q.shape
-        hkv = k.shape[1]
-        t = mask.total_seq_len
-        if nq != mask.q_len or k.shape[2] != t + nq or v.shape != k.shape:
-            raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match the mask "
-                             f"(T {t}, {mask.q_len} block rows)")
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        dev = q.device
-        out = torch.empty(1, nq, hq, d, device=dev, dtype=torch.bfloat16)
-        lse = torch.empty(hq, nq, device=dev, dtype=torch.float32)
-        nbytes = int(_lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 0))
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_fwd", q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), mask.ctx_lo, mask.ctx_hi,
-                  mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling),
-                  out, lse, ws, ws.numel(), _lib.stream_ptr(dev))
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.mask, ctx.scaling = mask, float(scaling)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse = ctx.saved_tensors
-        mask = ctx.mask
-        _, hq, nq, d = q.shape
-        hkv = k.shape[1]
-        t = mask.total_seq_len
-        dev = q.device
-        dout = dout.to(torch.bfloat16).contiguous()
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        nbytes = int(_lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 1))
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_bwd", q, q.stride(1), k, k.stride(1),
-                  v, v.stride(1), out, dout, lse,
-                  mask.ctx_lo, mask.ctx_hi, mask.blk_lo,
-                  mask.blk_hi, t, nq, hq, hkv, d, ctx.scaling, dq, dq.stride(1),
-                  dk, dk.stride(1), dv, dv.stride(1), ws, ws.numel(),
-                  _lib.stream_ptr(dev))
-        return dq, dk, dv, None, None
+def _dflash(q, k, v, mask: DFlashMask, scaling: float):
+    if q.dim() != 4 or q.shape[0] != 1:
+        raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, NQ, D]")
+    if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
+        raise _lib.SpxError("the HIP attention kernels take bf16 q/k/v")
+    t, nq = mask.total_seq_len, q.shape[2]
+    if nq != mask.q_len or k.shape[2] != t + nq or v.shape != k.shape:
+        raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match the mask "
+                         f"(T {t}, {mask.q_len} block rows)")
+    return _lib.native().attention(q, k, v, mask.ctx_lo, mask.ctx_hi, mask.blk_lo, mask.blk_hi, t, 0, scaling)
 
 
 def dflash_attention(q, k, v, mask: DFlashMask, scaling: float | None = None) -> torch.Tensor:
     """``[1, Hq, NQ, D]`` x ``[1, Hkv, T + NQ, D]`` -> ``[1, NQ, Hq, D]`` (bf16)."""
-    return _at_kernel_head_dim(_DFlashAttention.apply, q, k, v, mask, scaling)
+    return _at_kernel_head_dim(_dflash, q, k, v, mask, scaling)
 
 
 def dflash_hip_attention_forward(module, query, key, value, attention_mask, scaling=None, **_kwargs):

@@ -15,6 +15,7 @@
 #include <utility>
 
 #include "../../include/spx.h"
+#include "nodes.h"
 
 namespace {
 
@@ -122,12 +123,16 @@ PyObject* set_error(PyObject*, PyObject* cls) {
 #define SPX_VALUE(fn) SPX_ROW(fn)
 PyMethodDef g_methods[] = {
 #include "binding_list.h"
+    {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&spx_node_attention)), METH_FASTCALL, nullptr},
+    {"row_loss", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&spx_node_row_loss)), METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_spx_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
+
+PyObject* spx_error_class() { return g_error; }
 
 PyMODINIT_FUNC PyInit__spx_native() {
   g_error = PyExc_RuntimeError;

@@ -442,23 +442,23 @@ def fused_rows(op: int, logits, targets, target_stats=None, n_rows=None, step: S
 
 
 def kl_div_loss(logits, targets):
-    return fused_rows(OP_KL, logits, targets)[0]
+    return _lib.native().row_loss(OP_KL, logits, targets)
 
 
 def reverse_kl_div_loss(logits, targets):
-    return fused_rows(OP_RKL, logits, targets)[0]
+    return _lib.native().row_loss(OP_RKL, logits, targets)
 
 
 def js_div_loss(logits, targets):
-    return fused_rows(OP_JSD, logits, targets)[0]
+    return _lib.native().row_loss(OP_JSD, logits, targets)
 
 
 def ce_loss(logits, targets):
-    return fused_rows(OP_CE, logits, targets)[0]
+    return _lib.native().row_loss(OP_CE, logits, targets)
 
 
 def tv_loss(logits, targets):
-    return fused_rows(OP_TV, logits, targets)[0]
+    return _lib.native().row_loss(OP_TV, logits, targets)
 
 
 def neg_log_acceptance_loss(logits, targets):
