@@ -7,6 +7,8 @@
 // All exponentials run in the base-2 domain (v_exp_f32 is 2^x): logits are
 // pre-scaled by log2(e), statistics are converted back at the end.
 
+#include <algorithm>
+
 #include "loss_common.h"
 #include "../../include/spx.h"
 
@@ -44,6 +46,7 @@ __device__ __forceinline__ RowStats shuffle_xor(const RowStats& s, int m) {
   return o;
 }
 
+template <int WAVES>
 __device__ __forceinline__ float block_sum(float v, float* lds) {
   v = wave_sum(v);
   __syncthreads();
@@ -51,8 +54,20 @@ __device__ __forceinline__ float block_sum(float v, float* lds) {
   __syncthreads();
   float t = 0.f;
 #pragma unroll
-  for (int w = 0; w < kLossWaves; ++w) t += lds[w];
+  for (int w = 0; w < WAVES; ++w) t += lds[w];
   return t;
+}
+// merges the statistics of all threads; every thread gets the result
+template <int WAVES>
+__device__ __forceinline__ RowStats block_merge(RowStats s, RowStats* part) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) merge(s, shuffle_xor(s, m));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = part[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) merge(s, part[w]);
+  return s;
 }
 
 // log((2^a' + 2^b')/2) in natural units from natural-log inputs
@@ -104,13 +119,151 @@ __device__ __forceinline__ void load8_gather(const T* full, const int64_t* __res
   }
 }
 
+// eight elements of both rows into a thread's statistics
+template <int OP, bool KNOWN>
+__device__ __forceinline__ void add_chunk(RowStats& s, const float (&x)[8], const float (&y)[8], int64_t base,
+                                          float lt2_known) {
+      float cx = x[0], cy = y[0];
+  #pragma unroll
+      for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
+      if (!KNOWN) {
+  #pragma unroll
+        for (int i = 1; i < 8; ++i) cy = fmaxf(cy, y[i]);
+      }
+      if (cx > s.bd) {  // strict: an earlier chunk of this thread keeps a tie
+        int k = 7;
+  #pragma unroll
+        for (int i = 6; i >= 0; --i) k = (x[i] == cx) ? i : k;
+        s.bd = cx; s.id = (int)base + k;
+      }
+      if (!KNOWN && cy > s.bt) {
+        int k = 7;
+        float xv = x[7];
+  #pragma unroll
+        for (int i = 6; i >= 0; --i) {
+          const bool hit = y[i] == cy;
+          k = hit ? i : k;
+          xv = hit ? x[i] : xv;
+        }
+        s.bt = cy; s.it = (int)base + k; s.xt = xv;
+      }
+      {
+        const float cxs = cx * kLog2e;
+        float mn = s.md, z = s.zd;
+        if (cxs > mn) {  // the running max moves rarely once a few chunks have been seen
+          z *= fast_exp2(mn - cxs);
+          mn = cxs;
+        }
+  #pragma unroll
+        for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -mn));
+        s.zd = z; s.md = mn;
+      }
+      if (KNOWN && OP != SPX_LOSS_CE) {
+        float a = s.at;
+  #pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float pr = fast_exp2(fmaf(y[i], kLog2e, -lt2_known));  // the target probability
+          a = fmaf(pr, y[i] - x[i], a);
+        }
+        s.at = a;
+      } else if (OP != SPX_LOSS_CE) {
+        float mn = fmaxf(s.mt, cy * kLog2e);
+        float rs = fast_exp2(s.mt - mn);
+        float z = s.zt * rs, a = s.at * rs;
+  #pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          float e = fast_exp2(fmaf(y[i], kLog2e, -mn));
+          z += e;
+          if (OP == SPX_LOSS_KL) a = fmaf(e, y[i] - x[i], a);
+        }
+        s.zt = z; s.at = a; s.mt = mn;
+      }
+}
+
+// what the second pass over a row adds: rkl, jsd, tv
+template <int OP>
+__device__ __forceinline__ void add_second(float& acc, float& ext, const float (&x)[8], const float (&y)[8], float lse_d,
+                                           float lse_t) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float ldp = x[i] - lse_d, ltp = y[i] - lse_t;
+    float dp = fast_exp2(ldp * kLog2e), tp = fast_exp2(ltp * kLog2e);
+    if (OP == SPX_LOSS_RKL) {
+      acc = fmaf(dp, ldp - ltp, acc);
+    } else if (OP == SPX_LOSS_JSD) {
+      float lm = log_mix(ldp, ltp);
+      acc = fmaf(dp, ldp - lm, acc);
+      ext = fmaf(tp, ltp - lm, ext);
+    } else {  // TV
+      acc += fminf(dp, tp);
+      ext += (dp <= tp) ? dp : 0.f;
+    }
+  }
+}
+
+// one thread writes what a row leaves behind
+template <bool KNOWN>
+__device__ __forceinline__ void store_row(int64_t r, const RowStats& s, float row_loss, float lse_d, float row_extra,
+                                          float lse_t, float* __restrict__ loss, float* __restrict__ lse_draft,
+                                          float* __restrict__ lse_target, float* __restrict__ extra,
+                                          int32_t* __restrict__ argmax_draft, int32_t* __restrict__ argmax_target,
+                                          const StepArgs& sa) {
+  loss[r] = row_loss;
+  lse_draft[r] = lse_d;
+  extra[r] = row_extra;
+  if (argmax_draft) argmax_draft[r] = s.id;
+  if (!KNOWN) {
+    lse_target[r] = lse_t;
+    if (argmax_target) argmax_target[r] = s.it;
+  }
+  if (sa.counts) {
+    const bool m = sa.mask ? mask_value(sa.mask, sa.mask_kind, r) != 0.f : true;
+    const bool was = sa.prev ? mask_value(sa.prev, sa.prev_kind, r) != 0.f : true;
+    const bool now = was && (s.id == s.it);
+    if (m && now) atomicAdd(&sa.counts[0], 1);
+    if (m) atomicAdd(&sa.counts[1], 1);
+    if (was) atomicAdd(&sa.counts[2], 1);
+    if (sa.prev) store_flag(sa.prev, sa.prev_kind, r, now);
+  }
+}
+
 // ---- forward ---------------------------------------------------------------
 // KNOWN: lse_target / argmax_target are INPUTS (the target row's statistics from an
 // earlier pass over the same row); the target max / sum / arg-max tracking is skipped and
 // the cross-entropy reduction does not read the target row at all.
 // GATHER: the target row is read through the d2t offset table (see StepArgs).
-template <typename T, int OP, bool VEC, bool KNOWN, bool GATHER>
-__global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
+// eight elements as they come from memory
+template <typename T>
+struct RawChunk;
+template <>
+struct RawChunk<uint16_t> {
+  u32x4 a;
+  // KEEP: the row is read again, from L2
+  template <bool KEEP>
+  __device__ __forceinline__ void load(const uint16_t* p) { a = KEEP ? *reinterpret_cast<const u32x4*>(p) : ld16(p); }
+  __device__ __forceinline__ void get(float (&v)[8]) const {
+    v[0] = bf16_lo(a.x); v[1] = bf16_hi(a.x); v[2] = bf16_lo(a.y); v[3] = bf16_hi(a.y);
+    v[4] = bf16_lo(a.z); v[5] = bf16_hi(a.z); v[6] = bf16_lo(a.w); v[7] = bf16_hi(a.w);
+  }
+};
+template <>
+struct RawChunk<float> {
+  u32x4 a, b;
+  template <bool KEEP>
+  __device__ __forceinline__ void load(const float* p) {
+    a = KEEP ? *reinterpret_cast<const u32x4*>(p) : ld16(p);
+    b = KEEP ? *reinterpret_cast<const u32x4*>(p + 4) : ld16(p + 4);
+  }
+  __device__ __forceinline__ void get(float (&v)[8]) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[i] = __uint_as_float(a[i]); v[4 + i] = __uint_as_float(b[i]); }
+  }
+};
+
+constexpr int gather_stage_bytes(int threads) { return threads * 128; }
+// NT: threads per row.  A call of few rows leaves compute units idle with 256 (see fwd_threads).
+template <typename T, int OP, bool VEC, bool KNOWN, bool GATHER, int NT>
+__global__ __launch_bounds__(NT) void loss_fwd_kernel(
     const T* __restrict__ logits, int64_t ld_logits, const T* __restrict__ targets,
     int64_t ld_targets, int64_t vocab, float* __restrict__ loss, float* __restrict__ lse_draft,
     float* __restrict__ lse_target, float* __restrict__ extra, int32_t* __restrict__ argmax_draft,
@@ -132,10 +285,37 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
   // The span is brought into LDS with coalesced 16-byte loads and the eight elements of a lane
   // are picked from there; a span that does not fit (or rows without 16-byte alignment) and any
   // id that falls outside the span (a table that is not ascending) read the row directly.
-  constexpr int kStageElems = GATHER ? 32768 / (int)sizeof(T) : 1;
-  __shared__ __attribute__((aligned(16))) T stage[kStageElems];
-  for (int64_t c0 = 0; c0 < nchunks; c0 += kLossThreads) {
+  constexpr int kStageElems = GATHER ? gather_stage_bytes(NT) / (int)sizeof(T) : 1;
+  extern __shared__ __attribute__((aligned(16))) uint8_t stage_mem[];
+  T* const stage = reinterpret_cast<T*>(stage_mem);
+  // Without the gather: four chunks of each row are requested before the first is worked on (a row of 32000 is 16 trips of
+  // 256 threads, each of which waited a memory latency).
+  constexpr bool kStream = VEC && !GATHER;
+  constexpr bool kTwice = OP == SPX_LOSS_RKL || OP == SPX_LOSS_JSD || OP == SPX_LOSS_TV;
+  constexpr int U = 4;
+  const int64_t nfull = vocab >> 3;
+  if (kStream)
+    for (int64_t c = tid; c < nfull; c += NT * U) {
+      RawChunk<T> xr[U], yr[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + u * NT < nfull) {
+          xr[u].template load<kTwice>(xrow + ((c + u * NT) << 3));
+          if (read_y) yr[u].template load<kTwice>(yrow + ((c + u * NT) << 3));
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + u * NT < nfull) {
+          float x[8], y[8] = {};
+          xr[u].get(x);
+          if (read_y) yr[u].get(y);
+          add_chunk<OP, KNOWN>(s, x, y, (c + u * NT) << 3, lt2_known);
+        }
+    }
+  // (streaming: what is left is an incomplete last chunk, in the thread whose turn it is)
+  for (int64_t c0 = kStream ? nfull / NT * NT : 0; c0 < nchunks; c0 += NT) {
     const int64_t c = c0 + tid;
+    if (kStream && c < nfull) continue;
     const bool active = c < nchunks;
     const int64_t base = c << 3;
     float x[8], y[8];
@@ -158,7 +338,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
           for (int i = 0; i < 8; ++i) jj[i] = base + i < vocab ? base + i + sa.d2t[base + i] : -1;
         }
       }
-      const int64_t i0 = c0 << 3, i1 = min(vocab, (c0 + kLossThreads) << 3) - 1;
+      const int64_t i0 = c0 << 3, i1 = min(vocab, (c0 + NT) << 3) - 1;
       int64_t lo = i0 + sa.d2t[i0], hi = i1 + sa.d2t[i1] + 1;
       lo = max((int64_t)0, min(lo, sa.vt)) & ~(int64_t)7;
       hi = max(lo, min(hi, sa.vt));
@@ -167,7 +347,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
                           ptr_aligned16(targets);
       if (staged) {
         __syncthreads();  // the previous tile's picks are done
-        for (int64_t e = (int64_t)tid * EPV; lo + e < hi; e += kLossThreads * EPV) {
+        for (int64_t e = (int64_t)tid * EPV; lo + e < hi; e += NT * EPV) {
           if (lo + e + EPV <= sa.vt)
             *reinterpret_cast<u32x4*>(&stage[e]) = ld16(yrow + lo + e);
           else
@@ -194,76 +374,15 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
       if (read_y) load8<T, VEC>(yrow, base, vocab, y);
     }
     if (!active) continue;
-    float cx = x[0], cy = y[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
-    if (!KNOWN) {
-#pragma unroll
-      for (int i = 1; i < 8; ++i) cy = fmaxf(cy, y[i]);
-    }
-    if (cx > s.bd) {  // strict: an earlier chunk of this thread keeps a tie
-      int k = 7;
-#pragma unroll
-      for (int i = 6; i >= 0; --i) k = (x[i] == cx) ? i : k;
-      s.bd = cx; s.id = (int)base + k;
-    }
-    if (!KNOWN && cy > s.bt) {
-      int k = 7;
-      float xv = x[7];
-#pragma unroll
-      for (int i = 6; i >= 0; --i) {
-        const bool hit = y[i] == cy;
-        k = hit ? i : k;
-        xv = hit ? x[i] : xv;
-      }
-      s.bt = cy; s.it = (int)base + k; s.xt = xv;
-    }
-    {
-      const float cxs = cx * kLog2e;
-      float mn = s.md, z = s.zd;
-      if (cxs > mn) {  // the running max moves rarely once a few chunks have been seen
-        z *= fast_exp2(mn - cxs);
-        mn = cxs;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -mn));
-      s.zd = z; s.md = mn;
-    }
-    if (KNOWN && OP != SPX_LOSS_CE) {
-      float a = s.at;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float pr = fast_exp2(fmaf(y[i], kLog2e, -lt2_known));  // the target probability
-        a = fmaf(pr, y[i] - x[i], a);
-      }
-      s.at = a;
-    } else if (OP != SPX_LOSS_CE) {
-      float mn = fmaxf(s.mt, cy * kLog2e);
-      float rs = fast_exp2(s.mt - mn);
-      float z = s.zt * rs, a = s.at * rs;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float e = fast_exp2(fmaf(y[i], kLog2e, -mn));
-        z += e;
-        a = fmaf(e, y[i] - x[i], a);
-      }
-      s.zt = z; s.at = a; s.mt = mn;
-    }
+    add_chunk<OP, KNOWN>(s, x, y, base, lt2_known);
   }
 
   // tail padding must never win an arg-max: padded values are kNegBig, and
   // a padded index only enters when cx == kNegBig > -inf on an all-padding
   // chunk, which cannot exist (every chunk holds at least one real element).
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) merge(s, shuffle_xor(s, m));
-
-  __shared__ RowStats part[kLossWaves];
-  __shared__ float red[kLossWaves];
-  if ((tid & 63) == 0) part[tid >> 6] = s;
-  __syncthreads();
-  s = part[0];
-#pragma unroll
-  for (int w = 1; w < kLossWaves; ++w) merge(s, part[w]);
+  __shared__ RowStats part[NT / 64];
+  __shared__ float red[NT / 64];
+  s = block_merge<NT / 64>(s, part);
 
   const float lse_d = (s.md + fast_log2(s.zd)) * kLn2;
   const float lse_t = KNOWN ? lse_target[r]
@@ -282,53 +401,42 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_kernel(
   } else {
     // second streaming pass (the row pair is L2 resident by now)
     float acc = 0.f, ext = 0.f;
-    for (int64_t c = tid; c < nchunks; c += kLossThreads) {
+    if (kStream)
+      for (int64_t c = tid; c < nfull; c += NT * U) {
+        RawChunk<T> xr[U], yr[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (c + u * NT < nfull) {
+            xr[u].template load<false>(xrow + ((c + u * NT) << 3));
+            yr[u].template load<false>(yrow + ((c + u * NT) << 3));
+          }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (c + u * NT < nfull) {
+            float x[8], y[8];
+            xr[u].get(x);
+            yr[u].get(y);
+            add_second<OP>(acc, ext, x, y, lse_d, lse_t);
+          }
+      }
+    for (int64_t c = kStream ? nfull / NT * NT + tid : tid; c < nchunks; c += NT) {
+      if (kStream && c < nfull) continue;
       const int64_t base = c << 3;
       float x[8], y[8];
       load8<T, VEC>(xrow, base, vocab, x);
       if (GATHER) load8_gather<T>(yrow, sa.d2t, base, vocab, sa.vt, y);
       else load8<T, VEC>(yrow, base, vocab, y);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float ldp = x[i] - lse_d, ltp = y[i] - lse_t;
-        float dp = fast_exp2(ldp * kLog2e), tp = fast_exp2(ltp * kLog2e);
-        if (OP == SPX_LOSS_RKL) {
-          acc = fmaf(dp, ldp - ltp, acc);
-        } else if (OP == SPX_LOSS_JSD) {
-          float lm = log_mix(ldp, ltp);
-          acc = fmaf(dp, ldp - lm, acc);
-          ext = fmaf(tp, ltp - lm, ext);
-        } else {  // TV
-          acc += fminf(dp, tp);
-          ext += (dp <= tp) ? dp : 0.f;
-        }
-      }
+      add_second<OP>(acc, ext, x, y, lse_d, lse_t);
     }
-    acc = block_sum(acc, red);
-    if (OP != SPX_LOSS_RKL) ext = block_sum(ext, red);
+    acc = block_sum<NT / 64>(acc, red);
+    if (OP != SPX_LOSS_RKL) ext = block_sum<NT / 64>(ext, red);
     if (OP == SPX_LOSS_RKL) { row_loss = acc; row_extra = acc; }
     else if (OP == SPX_LOSS_JSD) { row_loss = 0.5f * (acc + ext); row_extra = acc; }
     else { row_loss = 1.f - acc; row_extra = ext; }
   }
-  if (tid == 0) {
-    loss[r] = row_loss;
-    lse_draft[r] = lse_d;
-    extra[r] = row_extra;
-    if (argmax_draft) argmax_draft[r] = s.id;
-    if (!KNOWN) {
-      lse_target[r] = lse_t;
-      if (argmax_target) argmax_target[r] = s.it;
-    }
-    if (sa.counts) {
-      const bool m = sa.mask ? mask_value(sa.mask, sa.mask_kind, r) != 0.f : true;
-      const bool was = sa.prev ? mask_value(sa.prev, sa.prev_kind, r) != 0.f : true;
-      const bool now = was && (s.id == s.it);
-      if (m && now) atomicAdd(&sa.counts[0], 1);
-      if (m) atomicAdd(&sa.counts[1], 1);
-      if (was) atomicAdd(&sa.counts[2], 1);
-      if (sa.prev) store_flag(sa.prev, sa.prev_kind, r, now);
-    }
-  }
+  if (tid == 0)
+    store_row<KNOWN>(r, s, row_loss, lse_d, row_extra, lse_t, loss, lse_draft, lse_target, extra, argmax_draft,
+                     argmax_target, sa);
 }
 
 // ---- forward and logits gradient in one pass -------------------------------------------------------
@@ -785,6 +893,8 @@ __global__ __launch_bounds__(kLossThreads) void loss_bwd_kernel(
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t nchunks = (vocab + 7) >> 3;
+  // (several workgroups share a row where there are few rows: blockIdx.y)
+  const int64_t c_first = (int64_t)blockIdx.y * kLossThreads + tid, c_stride = (int64_t)gridDim.y * kLossThreads;
   // with a row map the gradient of row r goes to row row_map[r] and rows mapped to -1 (zero gradient)
   // are not written: the live rows packed to the front
   int64_t dst = r;
@@ -797,7 +907,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_bwd_kernel(
   if (scale) g *= *scale;
   if (g == 0.f) {
     const float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int64_t c = tid; c < nchunks; c += kLossThreads) store8<T, VEC>(grow, c << 3, vocab, z);
+    for (int64_t c = c_first; c < nchunks; c += c_stride) store8<T, VEC>(grow, c << 3, vocab, z);
     return;
   }
   const T* xrow = logits + r * ld_logits;
@@ -808,26 +918,12 @@ __global__ __launch_bounds__(kLossThreads) void loss_bwd_kernel(
   const int label = (OP == SPX_LOSS_CE) ? argmax_target[r] : -1;
   const float cd = -lse_d * kLog2e, ct = -lse_t * kLog2e;
 
-#define SPX_LOSS_BWD_UNROLL 1
-  constexpr int UNR = SPX_LOSS_BWD_UNROLL;
-  for (int64_t c0 = tid; c0 < nchunks; c0 += kLossThreads * UNR) {
-    float xs[UNR][8], ys[UNR][8];
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int64_t c = c0 + (int64_t)u * kLossThreads;
-      if (c < nchunks) {
-        load8<T, VEC>(xrow, c << 3, vocab, xs[u]);
-        if (OP != SPX_LOSS_CE) load8<T, VEC>(yrow, c << 3, vocab, ys[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-    const int64_t c = c0 + (int64_t)u * kLossThreads;
-    if (c >= nchunks) break;
+  for (int64_t c = c_first; c < nchunks; c += c_stride) {
     const int64_t base = c << 3;
+    float x[8], y[8];
+    load8<T, VEC>(xrow, base, vocab, x);
+    if (OP != SPX_LOSS_CE) load8<T, VEC>(yrow, base, vocab, y);
     float o[8];
-    float* x = xs[u];
-    float* y = ys[u];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if (OP == SPX_LOSS_CE) {
@@ -848,7 +944,6 @@ __global__ __launch_bounds__(kLossThreads) void loss_bwd_kernel(
       }
     }
     store8<T, VEC>(grow, base, vocab, o);
-    }
   }
 }
 
@@ -1030,21 +1125,39 @@ __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
 // ---- dispatch ----------------------------------------------------------------
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <typename T, bool VEC, bool KNOWN, bool GATHER>
-static void launch_fwd(int op, const T* lg, int64_t ldl, const T* tg, int64_t ldt, int64_t rows,
-                       int64_t vocab, float* loss, float* lsd, float* lst, float* ex, int32_t* ad,
-                       int32_t* at, const StepArgs& sa, hipStream_t st) {
-  dim3 grid((unsigned)rows), block(kLossThreads);
-#define SPX_FWD(OPV)                                                                                 \
-  case OPV:                                                                                          \
-    hipLaunchKernelGGL((loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER>), grid, block, 0, st, lg, ldl,   \
-                       tg, ldt, vocab, loss, lsd, lst, ex, ad, at, sa);                              \
-    break;
+// Threads per row: enough that few rows fill the chip (2048 threads per compute unit), not so many that a compute unit holds
+// one row only and waits between them.  It depends on the rows alone: the gathering form of a call adds in the same order
+// and gives the same bits, except that above 64 rows its KL / CE form stays with the pipelined kernel of 256 threads.
+// Measured with 256 threads, a load at a time -> now (us), bf16: KL 64 rows of 128256 76 -> 26, 333 rows of 128256 92 -> 45, of
+// 32000 27 -> 17, 1024 of 32000 33 -> 28; TV 333 rows of 128256 171 -> 74; backward (columns over several workgroups) 64 rows of
+// 128256 66 -> 9.  (The row pair held in the registers of 1024 threads, so that the second pass reads no memory, was slower:
+// one workgroup per compute unit, 277 -> 160 us for RKL over 4096 rows of 32000 the other way.)
+static int threads_per_row(int64_t rows) { return rows <= 256 ? 1024 : rows <= 512 ? 512 : kLossThreads; }
+
+template <typename T, bool VEC, bool KNOWN, bool GATHER, int NT>
+static int launch_fwd(const char* fname, int op, const T* lg, int64_t ldl, const T* tg, int64_t ldt, int64_t rows,
+                      int64_t vocab, float* loss, float* lsd, float* lst, float* ex, int32_t* ad,
+                      int32_t* at, const StepArgs& sa, hipStream_t st) {
+  const dim3 grid((unsigned)rows), block(NT);
+  constexpr int lds = GATHER ? gather_stage_bytes(NT) : 0;
+#define SPX_FWD(OPV)                                                                                               \
+  case OPV: {                                                                                                      \
+    if constexpr (lds > 65536) {                                                                                   \
+      static std::atomic<uint64_t> lds_set;                                                                        \
+      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER, NT>), \
+                                      lds, lds_set, fname))                                                        \
+        return rc;                                                                                                 \
+    }                                                                                                              \
+    hipLaunchKernelGGL((loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER, NT>), grid, block, lds, st, lg, ldl, tg, ldt,  \
+                       vocab, loss, lsd, lst, ex, ad, at, sa);                                                     \
+    break;                                                                                                         \
+  }
   switch (op) {
     SPX_FWD(SPX_LOSS_KL) SPX_FWD(SPX_LOSS_RKL) SPX_FWD(SPX_LOSS_JSD) SPX_FWD(SPX_LOSS_CE)
     SPX_FWD(SPX_LOSS_TV)
   }
 #undef SPX_FWD
+  return check_launch(fname);
 }
 
 template <typename T, bool VEC>
@@ -1052,7 +1165,9 @@ static void launch_bwd(int op, const T* lg, int64_t ldl, const T* tg, int64_t ld
                        int64_t vocab, const float* lsd, const float* lst, const float* ex,
                        const int32_t* at, const float* rg, const float* sc, T* grad, int64_t ldg,
                        const int32_t* row_map, hipStream_t st) {
-  dim3 grid((unsigned)rows), block(kLossThreads);
+  // at least 2048 workgroups, each with a chunk per thread
+  const int64_t parts = std::max<int64_t>(1, std::min((2048 + rows - 1) / rows, (vocab / 8 + kLossThreads - 1) / kLossThreads));
+  dim3 grid((unsigned)rows, (unsigned)parts), block(kLossThreads);
 #define SPX_BWD(OPV)                                                                         \
   case OPV:                                                                                  \
     hipLaunchKernelGGL((loss_bwd_kernel<T, OPV, VEC>), grid, block, 0, st, lg, ldl, tg, ldt, \
@@ -1107,7 +1222,8 @@ static int loss_fwd_impl(const char* fname, int op, const void* logits, int64_t 
                    (gather ? (!sa.gathered || (aligned16(sa.gathered) && sa.ld_gathered % per16 == 0))
                            : (no_targets || (aligned16(targets) && ld_targets % per16 == 0)));
   // the first step of the verifier-logits entry in its common form: the pipelined kernel
-  if (gather && vec && dtype == SPX_DTYPE_BF16 && (op == SPX_LOSS_KL || op == SPX_LOSS_CE) &&
+  const int nt = threads_per_row(rows);
+  if (gather && vec && (nt == kLossThreads || rows > 64) && dtype == SPX_DTYPE_BF16 && (op == SPX_LOSS_KL || op == SPX_LOSS_CE) &&
       aligned16(targets) && ld_targets % 8 == 0 && vocab <= (int64_t)kPipeMaxTiles * kPipeTileIds &&
       sa.vt < (1ll << 30)) {
     static std::atomic<uint64_t> lds_set[2];  // per instantiation, one bit per device
@@ -1126,10 +1242,16 @@ static int loss_fwd_impl(const char* fname, int op, const void* logits, int64_t 
                          ld_targets, vocab, loss, lse_draft, lse_target, extra, argmax_draft, argmax_target, sa);
     return check_launch(fname);
   }
-#define SPX_GO(TT, VV, KK, GG)                                                                    \
-  launch_fwd<TT, VV, KK, GG>(op, reinterpret_cast<const TT*>(logits), ld_logits,                  \
-                             reinterpret_cast<const TT*>(targets), ld_targets, rows, vocab, loss, \
-                             lse_draft, lse_target, extra, argmax_draft, argmax_target, sa, st)
+#define SPX_GO_N(TT, VV, KK, GG, NN)                                                                        \
+  return launch_fwd<TT, VV, KK, GG, NN>(fname, op, reinterpret_cast<const TT*>(logits), ld_logits,           \
+                                        reinterpret_cast<const TT*>(targets), ld_targets, rows, vocab, loss, \
+                                        lse_draft, lse_target, extra, argmax_draft, argmax_target, sa, st)
+#define SPX_GO(TT, VV, KK, GG)                                                                        \
+  do {                                                                                                \
+    if (nt == 1024) SPX_GO_N(TT, VV, KK, GG, 1024);                                                   \
+    else if (nt == 512) SPX_GO_N(TT, VV, KK, GG, 512);                                                \
+    else SPX_GO_N(TT, VV, KK, GG, kLossThreads);                                                      \
+  } while (0)
 #define SPX_GO_T(TT)                                                                   \
   do {                                                                                 \
     if (gather) { if (vec) SPX_GO(TT, true, false, true); else SPX_GO(TT, false, false, true); } \
@@ -1140,7 +1262,7 @@ static int loss_fwd_impl(const char* fname, int op, const void* logits, int64_t 
   else SPX_GO_T(float);
 #undef SPX_GO_T
 #undef SPX_GO
-  return check_launch(fname);
+#undef SPX_GO_N
 }
 
 extern "C" int spx_fused_vocab_loss_fwd(int op, const void* logits, int64_t ld_logits,
