@@ -45,12 +45,13 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits16) {
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// round-to-nearest-even fp32 -> bf16 bits (NaN kept quiet)
+// round-to-nearest-even fp32 -> bf16 bits (NaN kept quiet): v_cvt_pk_bf16_f32.  Written out in integer
+// instructions the test for NaN was a branch around every value, which made the kernels that round at
+// every step (norms, rotary embedding) bound by instructions at half the memory's rate.
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return u >> 16;
+  union { __bf16 b; uint16_t u; } c;
+  c.b = (__bf16)f;
+  return c.u;
 }
 // two fp32 -> packed bf16 pair with the gfx950 conversion instruction
 // (v_cvt_pk_bf16_f32, round-to-nearest-even)
