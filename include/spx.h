@@ -519,6 +519,22 @@ int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_stride, void
                  int32_t hq, int32_t hkv, int32_t D, int32_t rotary_dim, int32_t inverse,
                  int64_t position_offset, float table_scale, void* stream);
 
+/* Per-head RMSNorm (over D, gain [D]), rotary embedding (all of D) and relayout in one pass: head h < n_heads of token
+ * t is tok[t * ld_tok + h * D ...], its normed and rotated form goes to out[h * out_head_stride + t * D ...] and
+ * 1 / rms to rstd[t * n_heads + h]; the n_pass heads behind them are copied to pass.  The rounding points are those of
+ * spx_rmsnorm_fwd followed by spx_rope_relayout.  D in {64, 128, 256}.
+ * The backward writes dtok (the rows' gradient, the passed heads moved back) and the gain's partial sums,
+ * spx_rmsnorm_bwd_slots(T * n_heads, D) rows of D (dw_scratch, may be NULL; reduced by spx_rmsnorm_dweight). */
+int spx_head_norm_rope(const void* tok, int64_t ld_tok, void* out, int64_t out_head_stride, void* pass,
+                       int64_t pass_head_stride, const int64_t* position_ids, const float* inv_freq,
+                       const void* gain, float* rstd, int64_t T, int32_t n_heads, int32_t n_pass, int32_t D,
+                       int64_t position_offset, float table_scale, float eps, void* stream);
+int spx_head_norm_rope_bwd(const void* tok, int64_t ld_tok, const void* dout, int64_t dout_head_stride,
+                           const void* dpass, int64_t dpass_head_stride, const int64_t* position_ids,
+                           const float* inv_freq, const void* gain, const float* rstd, void* dtok,
+                           int64_t ld_dtok, float* dw_scratch, int32_t accumulate, int64_t T, int32_t n_heads,
+                           int32_t n_pass, int32_t D, int64_t position_offset, float table_scale, void* stream);
+
 /* Rotary embedding fused with the head-major relayout that precedes attention
  * (apply_rotary_pos_emb + the view/transpose of LlamaAttention.forward; for
  * DFlash models/dflash/model_definitions.py:29-45):

@@ -64,6 +64,9 @@ SIGNATURES["spx_rmsnorm_pair_bwd_partial"] = [_P, _I64, _P, _P, _I64, _P, _P, _I
                                               _I32, _P, _I32, _I64, _I64, _P]
 SIGNATURES["spx_rope_qkv"] = [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32,
                               _I64, _F, _P]
+SIGNATURES["spx_head_norm_rope"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I64, _F, _F, _P]
+SIGNATURES["spx_head_norm_rope_bwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I32, _I64, _I32, _I32,
+                                        _I32, _I64, _F, _P]
 SIGNATURES["spx_rmsnorm_bwd_slots"] = [_I64, _I64]
 SIGNATURES["spx_rmsnorm_bwd"] = [_P, _I64, _P, _P, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _P]
 SIGNATURES["spx_add_rmsnorm_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P, _I64, _I64, _F, _P]

@@ -300,7 +300,7 @@ def create_padding_span_mask(attention_mask: torch.Tensor) -> SpanMask:
                     b * n)
 
 
-def _span(q, k, v, mask: SpanMask, scaling: float):
+def _check_span(q, k, v, mask: SpanMask) -> int:
     if q.dim() != 4 or q.shape[0] != 1:
         raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, T, D]")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
@@ -309,6 +309,11 @@ def _span(q, k, v, mask: SpanMask, scaling: float):
     if t != mask.total_seq_len or k.shape[2] != t or v.shape != k.shape:
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match a span mask over "
                          f"{mask.total_seq_len} positions")
+    return t
+
+
+def _span(q, k, v, mask: SpanMask, scaling: float):
+    t = _check_span(q, k, v, mask)
     return _lib.native().attention(q, k, v, mask.row_lo, mask.row_hi, None, None, t, 0, scaling)
 
 
@@ -378,7 +383,7 @@ def create_dflash_mask(document_ids: torch.Tensor, total_seq_len: int,
     return DFlashMask(bounds[0], bounds[1], bounds[2], bounds[3], total_seq_len, n_q)
 
 
-def _dflash(q, k, v, mask: DFlashMask, scaling: float):
+def _check_dflash(q, k, v, mask: DFlashMask) -> int:
     if q.dim() != 4 or q.shape[0] != 1:
         raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, NQ, D]")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
@@ -387,6 +392,11 @@ def _dflash(q, k, v, mask: DFlashMask, scaling: float):
     if nq != mask.q_len or k.shape[2] != t + nq or v.shape != k.shape:
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match the mask "
                          f"(T {t}, {mask.q_len} block rows)")
+    return t
+
+
+def _dflash(q, k, v, mask: DFlashMask, scaling: float):
+    t = _check_dflash(q, k, v, mask)
     return _lib.native().attention(q, k, v, mask.ctx_lo, mask.ctx_hi, mask.blk_lo, mask.blk_hi, t, 0, scaling)
 
 
@@ -403,6 +413,59 @@ def dflash_hip_attention_forward(module, query, key, value, attention_mask, scal
             f"attention impl '{ATTN_IMPL_DFLASH}' needs a DFlashMask descriptor as attention_mask, "
             f"got {type(attention_mask).__name__}")
     return dflash_attention(query, key, value, attention_mask, scaling), None
+
+
+def masked_forward_into(q, k, v, mask, scaling: float, out) -> torch.Tensor:
+    """The forward kernel of any of the masks (a ``TTTMask`` at its first step) into ``out`` (``NQ * Hq * D``
+    contiguous bf16 elements); returns the row statistics."""
+    if isinstance(mask, TTTMask):
+        _check_qkv(q, k, v, mask)
+        return ttt_forward_into(q, k, v, mask, scaling, out)
+    t = _check_span(q, k, v, mask) if isinstance(mask, SpanMask) else _check_dflash(q, k, v, mask)
+    _, hq, nq, d = q.shape
+    hkv = k.shape[1]
+    dev = q.device
+    lse = torch.empty(hq, nq, device=dev, dtype=torch.float32)
+    if isinstance(mask, SpanMask):
+        nbytes = _workspace_bytes(nq, hq, hkv, d, False)
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _lib.call("spx_span_attn_fwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), mask.row_lo, mask.row_hi, nq,
+                  hq, hkv, d, float(scaling), out, lse, ws, nbytes, _lib.stream_ptr(dev))
+    else:
+        nbytes = _lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 0)
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _lib.call("spx_dflash_attn_fwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), mask.ctx_lo, mask.ctx_hi,
+                  mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling), out, lse, ws, nbytes,
+                  _lib.stream_ptr(dev))
+    return lse
+
+
+def masked_backward(q, k, v, out, dout, lse, mask, scaling: float):
+    """``(dq, dk, dv)`` of ``masked_forward_into``."""
+    _, hq, nq, d = q.shape
+    hkv = k.shape[1]
+    dev = q.device
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    st = _lib.stream_ptr(dev)
+    if isinstance(mask, DFlashMask):
+        t = mask.total_seq_len
+        nbytes = _lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 1)
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _lib.call("spx_dflash_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.ctx_lo,
+                  mask.ctx_hi, mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling), dq, dq.stride(1), dk,
+                  dk.stride(1), dv, dv.stride(1), ws, nbytes, st)
+        return dq, dk, dv
+    nbytes = _workspace_bytes(nq, hq, hkv, d, True)
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    if isinstance(mask, SpanMask):
+        _lib.call("spx_span_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo,
+                  mask.row_hi, nq, hq, hkv, d, float(scaling), dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1),
+                  ws, nbytes, st)
+    else:
+        _lib.call("spx_ttt_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo, nq,
+                  mask.ttt_step, hq, hkv, d, float(scaling), dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1), ws,
+                  nbytes, st)
+    return dq, dk, dv
 
 
 class AttentionRegistry(dict):

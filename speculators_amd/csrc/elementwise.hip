@@ -422,6 +422,195 @@ __global__ __launch_bounds__(256) void rope_qkv_kernel(uint16_t* __restrict__ to
   }
 }
 
+// ---------------------------------------------------------------- per-head RMSNorm + rotary embedding + relayout
+// Heads 0 .. n_heads - 1 of a token row (n_heads * D elements, head h at h * D) are normed over their D elements, rotated
+// and written head-major; the n_pass heads behind them are only moved (the values).  The rounding points are those of the
+// separate kernels: bf16(x * rstd), its product with the gain, each product and the sum of the rotation.  D / 16 lanes share
+// a head, each with the two chunks of eight that rotate together; a thread works on HEADS heads of one token and evaluates
+// the angles once.  Bound by HBM where the rows fill the chip; one read and one write of q and k where the norm and the
+// relayout made two each (16384 tokens, 16 + 2 heads of 256: 345 us -> 91, the way back 375 -> 120).
+template <int D, int HEADS>
+__global__ __launch_bounds__(256) void head_norm_rope_kernel(const uint16_t* __restrict__ tok, int64_t ld,
+                                                             uint16_t* __restrict__ out, int64_t hs_out,
+                                                             uint16_t* __restrict__ pass, int64_t hs_pass,
+                                                             const int64_t* __restrict__ pos,
+                                                             const float* __restrict__ inv_freq,
+                                                             const uint16_t* __restrict__ gain, float* __restrict__ rstd,
+                                                             int T, int n_heads, int n_pass, int64_t pos_offset,
+                                                             float table_scale, float eps) {
+  constexpr int L = D / 16;
+  const int heads = n_heads + n_pass, groups = (heads + HEADS - 1) / HEADS;
+  const int64_t item = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+  if (item >= (int64_t)T * groups) return;  // (all lanes of a head together)
+  const int hg = (int)(item % groups), t = (int)(item / groups);
+  const int part = threadIdx.x % L, d0 = part * 8;
+  u32x4 ra[HEADS], rb[HEADS];
+#pragma unroll
+  for (int i = 0; i < HEADS; ++i) {
+    const int h = i * groups + hg;
+    ra[i] = rb[i] = u32x4{0, 0, 0, 0};
+    if (h < heads) {
+      const uint16_t* src = tok + (int64_t)t * ld + h * D + d0;
+      ra[i] = *reinterpret_cast<const u32x4*>(src);
+      rb[i] = *reinterpret_cast<const u32x4*>(src + D / 2);
+    }
+  }
+  float c[8], s[8], wa[8], wb[8];
+  if (hg < n_heads) {
+    unpack8f(*reinterpret_cast<const u32x4*>(gain + d0), wa);
+    unpack8f(*reinterpret_cast<const u32x4*>(gain + D / 2 + d0), wb);
+    const float p = (float)(pos[t] + pos_offset);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float sn, cs;
+      sincosf(p * inv_freq[d0 + e], &sn, &cs);
+      c[e] = round_bf16(cs * table_scale);
+      s[e] = round_bf16(sn * table_scale);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < HEADS; ++i) {
+    const int h = i * groups + hg;
+    float a[8], b[8], ss = 0.f;
+    unpack8f(ra[i], a);
+    unpack8f(rb[i], b);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = fmaf(a[e], a[e], fmaf(b[e], b[e], ss));
+#pragma unroll
+    for (int m = 1; m < L; m <<= 1) ss += __shfl_xor(ss, m, 64);
+    if (h >= heads) continue;
+    uint16_t* dst;
+    if (h < n_heads) {
+      const float r = rsqrtf(ss / (float)D + eps);
+      if (part == 0) rstd[(int64_t)t * n_heads + h] = r;
+      float oa[8], ob[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        a[e] = round_bf16(wa[e] * round_bf16(a[e] * r));
+        b[e] = round_bf16(wb[e] * round_bf16(b[e] * r));
+        oa[e] = round_bf16(a[e] * c[e]) + round_bf16(-b[e] * s[e]);
+        ob[e] = round_bf16(b[e] * c[e]) + round_bf16(a[e] * s[e]);
+      }
+      ra[i] = pack8f(oa);
+      rb[i] = pack8f(ob);
+      dst = out + (int64_t)h * hs_out;
+    } else {
+      dst = pass + (int64_t)(h - n_heads) * hs_pass;
+    }
+    dst += (int64_t)t * D + d0;
+    *reinterpret_cast<u32x4*>(dst) = ra[i];
+    *reinterpret_cast<u32x4*>(dst + D / 2) = rb[i];
+  }
+}
+
+// The way back: dtok from the head-major gradients (rotated back, then through the norm), and the gain's partial sums, one
+// row of D per workgroup (slots as spx_rmsnorm_bwd_slots; accumulate: they start from what dw_part holds).
+template <int D, int HEADS>
+__global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(
+    const uint16_t* __restrict__ tok, int64_t ld, const uint16_t* __restrict__ dout, int64_t hs_out,
+    const uint16_t* __restrict__ dpass, int64_t hs_pass, const int64_t* __restrict__ pos,
+    const float* __restrict__ inv_freq, const uint16_t* __restrict__ gain, const float* __restrict__ rstd,
+    uint16_t* __restrict__ dtok, int64_t ld_d, float* __restrict__ dw_part, int accumulate, int T, int n_heads, int n_pass,
+    int64_t pos_offset, float table_scale) {
+  constexpr int L = D / 16, PER = 256 / L;
+  __shared__ float red[PER * D];
+  const int heads = n_heads + n_pass, groups = (heads + HEADS - 1) / HEADS;
+  const int part = threadIdx.x % L, d0 = part * 8;
+  const int64_t items = (int64_t)T * groups;
+  float wa[8], wb[8], dwa[8], dwb[8];
+  unpack8f(*reinterpret_cast<const u32x4*>(gain + d0), wa);
+  unpack8f(*reinterpret_cast<const u32x4*>(gain + D / 2 + d0), wb);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) dwa[e] = dwb[e] = 0.f;
+  for (int64_t item = (int64_t)blockIdx.x * PER + threadIdx.x / L; item < items; item += (int64_t)gridDim.x * PER) {
+    const int hg = (int)(item % groups), t = (int)(item / groups);
+    u32x4 ga[HEADS], gb[HEADS], xa[HEADS], xb[HEADS];
+    float r[HEADS];
+#pragma unroll
+    for (int i = 0; i < HEADS; ++i) {
+      const int h = i * groups + hg;
+      ga[i] = gb[i] = xa[i] = xb[i] = u32x4{0, 0, 0, 0};
+      r[i] = 0.f;
+      if (h < heads) {
+        const uint16_t* g = (h < n_heads ? dout + (int64_t)h * hs_out : dpass + (int64_t)(h - n_heads) * hs_pass) +
+                            (int64_t)t * D + d0;
+        ga[i] = *reinterpret_cast<const u32x4*>(g);
+        gb[i] = *reinterpret_cast<const u32x4*>(g + D / 2);
+        if (h < n_heads) {
+          const uint16_t* x = tok + (int64_t)t * ld + h * D + d0;
+          xa[i] = *reinterpret_cast<const u32x4*>(x);
+          xb[i] = *reinterpret_cast<const u32x4*>(x + D / 2);
+          r[i] = rstd[(int64_t)t * n_heads + h];
+        }
+      }
+    }
+    float c[8], s[8];
+    if (hg < n_heads) {
+      const float p = (float)(pos[t] + pos_offset);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float sn, cs;
+        sincosf(p * inv_freq[d0 + e], &sn, &cs);
+        c[e] = round_bf16(cs * table_scale);
+        s[e] = -round_bf16(sn * table_scale);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < HEADS; ++i) {
+      const int h = i * groups + hg;
+      if (h < n_heads) {  // (uniform over the lanes of a head)
+        float a[8], b[8], ha[8], hb[8], dot = 0.f;
+        unpack8f(ga[i], a);
+        unpack8f(gb[i], b);
+        unpack8f(xa[i], ha);
+        unpack8f(xb[i], hb);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          // the gradient of the norm's output, as the separate kernel would have stored it
+          const float da = round_bf16(round_bf16(a[e] * c[e]) + round_bf16(-b[e] * s[e]));
+          const float db = round_bf16(round_bf16(b[e] * c[e]) + round_bf16(a[e] * s[e]));
+          ha[e] *= r[i];
+          hb[e] *= r[i];
+          dwa[e] = fmaf(da, ha[e], dwa[e]);
+          dwb[e] = fmaf(db, hb[e], dwb[e]);
+          a[e] = da * wa[e];
+          b[e] = db * wb[e];
+          dot = fmaf(a[e], ha[e], fmaf(b[e], hb[e], dot));
+        }
+#pragma unroll
+        for (int m = 1; m < L; m <<= 1) dot += __shfl_xor(dot, m, 64);
+        const float mean = dot / (float)D;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          a[e] = r[i] * (a[e] - ha[e] * mean);
+          b[e] = r[i] * (b[e] - hb[e] * mean);
+        }
+        ga[i] = pack8f(a);
+        gb[i] = pack8f(b);
+      }
+      if (h < heads) {
+        uint16_t* dst = dtok + (int64_t)t * ld_d + h * D + d0;
+        *reinterpret_cast<u32x4*>(dst) = ga[i];
+        *reinterpret_cast<u32x4*>(dst + D / 2) = gb[i];
+      }
+    }
+  }
+  if (!dw_part) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    red[threadIdx.x / L * D + d0 + e] = dwa[e];
+    red[threadIdx.x / L * D + D / 2 + d0 + e] = dwb[e];
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float* const o = dw_part + (int64_t)blockIdx.x * D + threadIdx.x;
+    float sum = accumulate ? *o : 0.f;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) sum += red[k * D + threadIdx.x];
+    *o = sum;
+  }
+}
+
 // out[b][c][r] = in[b][r][c] for a stack of bf16 matrices (the per-expert transposes the input
 // gradient products of a stack of expert weights need).  One wave = one 64 x 64 tile, one lane =
 // one 8 x 8 block transposed in registers: every load and store instruction moves whole 128-byte
@@ -600,6 +789,8 @@ __global__ __launch_bounds__(256) void unpack_rows_kernel(const uint16_t* __rest
 }  // namespace spx
 
 using namespace spx;
+
+#define SPX_REQ_FN(cond, what) do { if (!(cond)) return spx::fail_arg(fn, what); } while (0)
 
 extern "C" int spx_pack_row_map(const float* row_grad, const int64_t* labels, int64_t ignore_index,
                                 int64_t rows, int32_t* row_map, int32_t* count, void* stream) {
@@ -849,7 +1040,6 @@ extern "C" int spx_rope_relayout_partial(const void* x, int64_t ld_x, int32_t x_
                             inverse, position_offset, x_head_stride, rotary_dim, table_scale, stream);
 }
 
-#define SPX_REQ_FN(cond, what) do { if (!(cond)) return spx::fail_arg(fn, what); } while (0)
 extern "C" int spx_transpose_bf16(const void* in, int64_t ld_in, int64_t batch_stride_in, void* out,
                                   int64_t ld_out, int64_t batch_stride_out, int64_t R, int64_t C,
                                   int64_t batches, void* stream) {
@@ -991,11 +1181,81 @@ extern "C" int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_s
 #undef SPX_LAUNCH
   return check_launch(fn);
 }
-#undef SPX_REQ_FN
 
 static unsigned swiglu_grid(int64_t n8) {
   return (unsigned)((n8 + 255) / 256 < 65536 ? (n8 + 255) / 256 : 65536);
 }
+
+static int head_norm_rope_checks(const char* fn, int64_t ld, int64_t T, int32_t n_heads, int32_t n_pass, int32_t D,
+                                 int64_t hs, int64_t hs_pass, float table_scale) {
+  SPX_REQ_FN(table_scale > 0.f && table_scale < 1e4f, "the table scale must be positive and finite");
+  SPX_REQ_FN(T > 0 && n_heads > 0 && n_pass >= 0, "T and heads must be positive");
+  SPX_REQ_FN(D == 64 || D == 128 || D == 256, "head_dim must be 64, 128 or 256");
+  SPX_REQ_FN(ld % 8 == 0 && ld >= (int64_t)(n_heads + n_pass) * D, "bad row stride of the token-major side");
+  SPX_REQ_FN(hs % 8 == 0 && hs >= T * D && (!n_pass || (hs_pass % 8 == 0 && hs_pass >= T * D)),
+             "head strides must be multiples of 8, at least T * D");
+  SPX_REQ_FN(T * (n_heads + n_pass) * (D / 16) < (1ll << 31), "too many elements");
+  return SPX_OK;
+}
+// heads per thread: as many as leave every compute unit two workgroups
+static int heads_per_thread(int64_t threads) { return threads >= 4 * 512 * 256 ? 4 : threads >= 2 * 512 * 256 ? 2 : 1; }
+
+extern "C" int spx_head_norm_rope(const void* tok, int64_t ld_tok, void* out, int64_t out_head_stride, void* pass,
+                                  int64_t pass_head_stride, const int64_t* position_ids, const float* inv_freq,
+                                  const void* gain, float* rstd, int64_t T, int32_t n_heads, int32_t n_pass, int32_t D,
+                                  int64_t position_offset, float table_scale, float eps, void* stream) {
+  const char* fn = __func__;
+  if (int rc = head_norm_rope_checks(fn, ld_tok, T, n_heads, n_pass, D, out_head_stride, pass_head_stride, table_scale))
+    return rc;
+  SPX_REQ_FN(tok && out && position_ids && inv_freq && gain && rstd && (!n_pass || pass), "null buffer");
+  SPX_REQ_FN(al16(tok) && al16(out) && al16(pass) && al16(gain), "buffers must be 16-byte aligned");
+  const int64_t threads = T * (n_heads + n_pass) * (D / 16);
+  const int per = heads_per_thread(threads);
+#define SPX_LAUNCH(DD, HEADS)                                                                                         \
+  hipLaunchKernelGGL((head_norm_rope_kernel<DD, HEADS>),                                                              \
+                     dim3((unsigned)((T * ((n_heads + n_pass + HEADS - 1) / HEADS) * (DD / 16) + 255) / 256)), dim3(256), \
+                     0, reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(tok), ld_tok,        \
+                     reinterpret_cast<uint16_t*>(out), out_head_stride, reinterpret_cast<uint16_t*>(pass),            \
+                     pass_head_stride, position_ids, inv_freq, reinterpret_cast<const uint16_t*>(gain), rstd, (int)T, \
+                     (int)n_heads, (int)n_pass, position_offset, table_scale, eps)
+#define SPX_LAUNCH_D(HEADS)                                                                                           \
+  do { if (D == 64) SPX_LAUNCH(64, HEADS); else if (D == 128) SPX_LAUNCH(128, HEADS); else SPX_LAUNCH(256, HEADS); } while (0)
+  if (per == 4) SPX_LAUNCH_D(4);
+  else if (per == 2) SPX_LAUNCH_D(2);
+  else SPX_LAUNCH_D(1);
+#undef SPX_LAUNCH
+  return check_launch(fn);
+}
+
+extern "C" int spx_head_norm_rope_bwd(const void* tok, int64_t ld_tok, const void* dout, int64_t dout_head_stride,
+                                      const void* dpass, int64_t dpass_head_stride, const int64_t* position_ids,
+                                      const float* inv_freq, const void* gain, const float* rstd, void* dtok,
+                                      int64_t ld_dtok, float* dw_scratch, int32_t accumulate, int64_t T, int32_t n_heads,
+                                      int32_t n_pass, int32_t D, int64_t position_offset, float table_scale,
+                                      void* stream) {
+  const char* fn = __func__;
+  if (int rc = head_norm_rope_checks(fn, ld_tok, T, n_heads, n_pass, D, dout_head_stride, dpass_head_stride, table_scale))
+    return rc;
+  SPX_REQ_FN(tok && dout && position_ids && inv_freq && gain && rstd && dtok && (!n_pass || dpass), "null buffer");
+  SPX_REQ_FN(al16(tok) && al16(dout) && al16(dpass) && al16(gain) && al16(dtok), "buffers must be 16-byte aligned");
+  SPX_REQ_FN(ld_dtok % 8 == 0 && ld_dtok >= (int64_t)(n_heads + n_pass) * D, "bad row stride of the gradient");
+  const int64_t slots = spx_rmsnorm_bwd_slots(T * n_heads, D);
+  const int per = heads_per_thread(T * (n_heads + n_pass) * (D / 16));
+#define SPX_LAUNCH(DD, HEADS)                                                                                         \
+  hipLaunchKernelGGL((head_norm_rope_bwd_kernel<DD, HEADS>), dim3((unsigned)slots), dim3(256), 0,                     \
+                     reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(tok), ld_tok,           \
+                     reinterpret_cast<const uint16_t*>(dout), dout_head_stride,                                       \
+                     reinterpret_cast<const uint16_t*>(dpass), dpass_head_stride, position_ids, inv_freq,             \
+                     reinterpret_cast<const uint16_t*>(gain), rstd, reinterpret_cast<uint16_t*>(dtok), ld_dtok,       \
+                     dw_scratch, (int)accumulate, (int)T, (int)n_heads, (int)n_pass, position_offset, table_scale)
+  if (per >= 2) SPX_LAUNCH_D(2);
+  else SPX_LAUNCH_D(1);
+#undef SPX_LAUNCH
+#undef SPX_LAUNCH_D
+  return check_launch(fn);
+}
+
+#undef SPX_REQ_FN
 
 extern "C" int spx_swiglu_rows_fwd(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up,
                                    void* out, int64_t ld_out, int64_t rows, int64_t F, void* stream) {

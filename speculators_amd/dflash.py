@@ -24,6 +24,7 @@ from torch import nn
 from . import attention as A
 from . import fused_ops as FO
 from . import gemm
+from . import layer as LY
 from . import losses as L
 from . import metrics as MT
 from .eagle3 import MLP, RMSNorm
@@ -120,9 +121,24 @@ class DFlashDecoderLayer(nn.Module):
     def __init__(self, cfg: DFlashConfig, stager: WeightStager):
         super().__init__()
         self.self_attn = DFlashAttention(cfg, stager)
+        self._stager = stager
         self.mlp = MLP(cfg, stager)
         self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, stager)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, stager)
+
+    def _step(self, q_pos, kv_pos, inv_freq, mask, next_norm):
+        """The layer as one node (``layer.NormedLayer``), or None where it is put together from its parts: another
+        attention function or head size, or a graph in which some projection does not train."""
+        att = self.self_attn
+        if next_norm is None or not LY.NormedLayer.takes(att, inv_freq, A.dflash_hip_attention_forward):
+            return None
+        W = self._stager.get
+        ws = (W(att.q_proj.weight), W(att.k_proj.weight, att.v_proj.weight), W(att.o_proj.weight),
+              W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight), W(self.mlp.down_proj.weight))
+        if torch.is_grad_enabled() and not all(w.trainable for w in ws):
+            return None
+        return LY.NormedLayer(*ws, (0.0, att.q_norm.eps, att.k_norm.eps, self.post_attention_layernorm.eps,
+                                    next_norm.eps), (att.hq, att.hkv, att.d), att.scaling, q_pos, kv_pos, inv_freq, mask)
 
     def forward(self, x, ctx, q_pos, kv_pos, inv_freq, mask, x_normed=None, next_norm=None):
         """``x_normed``: ``input_layernorm(x)`` when the previous layer already produced it;
@@ -130,6 +146,11 @@ class DFlashDecoderLayer(nn.Module):
         ``(out, next_norm(out))`` with the last residual add fused into that norm."""
         if x_normed is None:
             x_normed = self.input_layernorm(x)
+        step = self._step(q_pos, kv_pos, inv_freq, mask, next_norm)
+        if step is not None and x.dtype == x_normed.dtype == ctx.dtype == torch.bfloat16:
+            step.take_slots(x.shape[1])
+            att, post = self.self_attn, self.post_attention_layernorm
+            return LY.run_normed(step, x, x_normed, ctx, None, att.q_norm.gain, att.k_norm.gain, post.gain, next_norm.gain)
         a = self.self_attn(x_normed, ctx, q_pos, kv_pos, inv_freq, mask)
         post = self.post_attention_layernorm
         y, z = FO.add_rms_norm(x, a, post.gain, post.eps)  # residual add fused into the norm

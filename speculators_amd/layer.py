@@ -1,4 +1,4 @@
-"""One TTT step of a draft decoder layer as ONE autograd node.
+"""A draft decoder layer -- one TTT step of it, or one pass -- as ONE autograd node.
 
 The layer (models/eagle3/model_definitions.py:14-110) is nine launches forward and thirteen backward; as
 eight nodes of their own they cost more host time (a node's forward and backward 20 us, and the views,
@@ -71,6 +71,16 @@ def step_forward(s: LayerStep, a, b, gain_a, gain_b, gain_post, gain_next):
     k, v = s.cache.k[:, :, :n], s.cache.v[:, :, :n]
     att = _rows(slot_o, t, hq * d, dev)
     lse = A.ttt_forward_into(q, k, v, s.mask, s.scaling, att)
+    y, normed, tail = _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_next)
+    return y, normed, (a2, b2, rstd_in, xin, q, att, lse, *tail)
+
+
+def _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_next):
+    """What follows the attention: output projection, residual add and norm, MLP, residual add and the norm
+    that reads the layer's output."""
+    t, h = residual.shape
+    dev = residual.device
+    st = _lib.stream_ptr(dev)
     o = gemm._project(att, s.wo)
     stats = torch.empty(2, t, device=dev, dtype=torch.float32)
     mid = torch.empty(t, h, device=dev, dtype=torch.bfloat16)
@@ -86,7 +96,40 @@ def step_forward(s: LayerStep, a, b, gain_a, gain_b, gain_post, gain_next):
     y = torch.empty(t, h, device=dev, dtype=torch.bfloat16)
     normed = _rows(slot_next, t, h, dev)
     _lib.call("spx_add_rmsnorm_fwd", mid, h, m, h, y, h, gain_next, normed, h, stats[1], t, h, s.eps_next, st)
-    return y, normed, (a2, b2, rstd_in, xin, q, att, lse, mid, stats, z, gu, act, y)
+    return y, normed, (mid, stats, z, gu, act, y)
+
+
+def _tail_backward(s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads_next, needs, taken):
+    """``(gradient of the residual stream in front of the attention, gradient of att, of the two gains, tokens of
+    wo, wgu, wd)``."""
+    mid, stats, z, gu, act, y = tail
+    slot_o, slot_gu, slot_d = taken
+    t, h = y.shape
+    f = act.shape[1]
+    dev = y.device
+    st = _lib.stream_ptr(dev)
+    if dy is not None:
+        dy = _flat(dy).to(torch.bfloat16)
+    dm = _rows(s.wd.dy_slot(slot_d, t), t, h, dev)
+    d_next = None
+    if dn is not None:
+        d_next = FO._norm_backward(grads_next, needs[1], y, gain_next, _flat(dn).to(torch.bfloat16), dy, stats[1],
+                                   dm, t, h)
+    else:
+        dm.copy_(dy)
+    dact = gemm._project_back(dm, s.wd)
+    tok_d = s.wd.defer(slot_d, dm, act)
+    dgu = _rows(s.wgu.dy_slot(slot_gu, t), t, 2 * f, dev)
+    base, dbase = gu.data_ptr(), dgu.data_ptr()
+    _lib.call("spx_swiglu_rows_bwd", base, 2 * f, base + 2 * f, 2 * f, dact, f, dbase, 2 * f, dbase + 2 * f, 2 * f,
+              t, f, st)
+    dz = gemm._project_back(dgu, s.wgu)
+    tok_gu = s.wgu.defer(slot_gu, dgu, z)
+    da = _rows(s.wo.dy_slot(slot_o, t), t, h, dev)
+    d_post = FO._norm_backward(grads_post, needs[0], mid, gain_post, dz, dm, stats[0], da, t, h)
+    datt = gemm._project_back(da, s.wo)
+    tok_o = s.wo.defer(slot_o, da, att)
+    return da, datt, d_post, d_next, tok_o, tok_gu, tok_d
 
 
 class _LayerStep(torch.autograd.Function):
@@ -116,33 +159,13 @@ class _LayerStep(torch.autograd.Function):
          gain_a, gain_b, gain_post, gain_next) = ctx.saved_tensors
         s = ctx.step
         needs = ctx.needs_input_grad
-        t, h = y.shape
-        f = act.shape[1]
+        t = y.shape[0]
         dev = y.device
-        st = _lib.stream_ptr(dev)
-        slot_qkv, slot_o, slot_gu, slot_d = ctx.taken
+        slot_qkv = ctx.taken[0]
         grads_a, grads_b, grads_post, grads_next = ctx.gain_grads
-        if dy is not None:
-            dy = _flat(dy).to(torch.bfloat16)
-        dm = _rows(s.wd.dy_slot(slot_d, t), t, h, dev)
-        d_next = None
-        if dn is not None:
-            d_next = FO._norm_backward(grads_next, needs[6], y, gain_next, _flat(dn).to(torch.bfloat16), dy, stats[1],
-                                       dm, t, h)
-        else:
-            dm.copy_(dy)
-        dact = gemm._project_back(dm, s.wd)
-        tok_d = s.wd.defer(slot_d, dm, act)
-        dgu = _rows(s.wgu.dy_slot(slot_gu, t), t, 2 * f, dev)
-        base, dbase = gu.data_ptr(), dgu.data_ptr()
-        _lib.call("spx_swiglu_rows_bwd", base, 2 * f, base + 2 * f, 2 * f, dact, f, dbase, 2 * f, dbase + 2 * f, 2 * f,
-                  t, f, st)
-        dz = gemm._project_back(dgu, s.wgu)
-        tok_gu = s.wgu.defer(slot_gu, dgu, z)
-        da = _rows(s.wo.dy_slot(slot_o, t), t, h, dev)
-        d_post = FO._norm_backward(grads_post, needs[5], mid, gain_post, dz, dm, stats[0], da, t, h)
-        datt = gemm._project_back(da, s.wo)
-        tok_o = s.wo.defer(slot_o, da, att)
+        da, datt, d_post, d_next, tok_o, tok_gu, tok_d = _tail_backward(
+            s, dy, dn, att, (mid, stats, z, gu, act, y), gain_post, gain_next, grads_post, grads_next, needs[5:7],
+            ctx.taken[1:])
         step_no = s.offset + 1
         k, v = s.cache.k[:, :, :step_no * t], s.cache.v[:, :, :step_no * t]
         dq, dk, dv = A.ttt_backward_shared(s.cache.grads, q, k, v, att, datt, lse, s.mask, step_no, s.scaling)
@@ -171,3 +194,172 @@ def run(s: LayerStep, a, b, gain_a, gain_b, gain_post, gain_next):
                                 s.wd.token)
     y, normed, _ = step_forward(s, a, b, gain_a, gain_b, gain_post, gain_next)
     return y.view(a.shape), normed.view(a.shape)
+
+
+class NormedLayer:
+    """A layer with per-head q / k norms over one set of keys.  The anchored-block draft's projects q from the
+    normed input (``wq``) and k, v from ``cat([context, normed input])`` (``wkv``); the multi-token-prediction
+    layer's does its own input norm and projects all three from it (``wqkv`` in the place of ``wq``)."""
+
+    __slots__ = ("wq", "wkv", "wo", "wgu", "wd", "eps_in", "eps_q", "eps_k", "eps_post", "eps_next", "hq", "hkv", "d",
+                 "scaling", "q_pos", "kv_pos", "inv_freq", "mask", "slots", "grad_slot")
+
+    def __init__(self, wq, wkv, wo, wgu, wd, eps, heads, scaling, q_pos, kv_pos, inv_freq, mask):
+        self.wq, self.wkv, self.wo, self.wgu, self.wd = wq, wkv, wo, wgu, wd
+        self.eps_in, self.eps_q, self.eps_k, self.eps_post, self.eps_next = eps
+        self.hq, self.hkv, self.d = heads
+        self.scaling, self.q_pos, self.kv_pos, self.inv_freq, self.mask = scaling, q_pos, kv_pos, inv_freq, mask
+        self.slots, self.grad_slot = (None,) * 4, None
+
+    @staticmethod
+    def takes(attention, inv_freq, kernel) -> bool:
+        """Whether ``attention`` is one the node's kernels serve (a head size they are built for, the rotary
+        embedding over all of it, the attention function ``kernel``)."""
+        d = attention.d
+        return attention.attn_fn is kernel and d in A.KERNEL_HEAD_DIMS and 2 * inv_freq.numel() == d
+
+    def tokens(self):
+        return tuple(w.token for w in (self.wq, self.wkv, self.wo, self.wgu, self.wd) if w is not None)
+
+    def take_slots(self, t: int):
+        """See ``LayerStep.take_slots``."""
+        self.slots = (self.wq.x_slot(t) if self.wkv is None else None, self.wo.x_slot(t), self.wgu.x_slot(t),
+                      self.wd.x_slot(t))
+
+
+def _head_norm_rope(tok, ld, out, passed, pos, s, gain, eps, t, heads, n_pass):
+    rstd = torch.empty(t, heads, device=out.device, dtype=torch.float32)
+    _lib.call("spx_head_norm_rope", tok, ld, out, t * s.d, passed, t * s.d, pos, s.inv_freq, gain, rstd, t, heads,
+              n_pass, s.d, 0, FO.table_scale_of(s.inv_freq), eps, _lib.stream_ptr(out.device))
+    return rstd
+
+
+def _head_norm_rope_backward(tok, ld, dout, dpass, pos, s, gain, rstd, grads, need_dw, dtok, ld_d, t, heads, n_pass):
+    """Writes ``dtok``; returns what autograd gets for the gain."""
+    dev = dout.device
+    st = _lib.stream_ptr(dev)
+    rows = t * heads
+    scratch, acc, shared = None, 0, None
+    if need_dw:
+        shared = grads.target(rows, s.d, dev) if grads is not None else None
+        scratch, acc = shared if shared is not None else (FO._dw_buffers(rows, s.d, dev)[0], 0)
+    _lib.call("spx_head_norm_rope_bwd", tok, ld, dout, t * s.d, dpass, t * s.d, pos, s.inv_freq, gain, rstd, dtok, ld_d,
+              scratch, acc, t, heads, n_pass, s.d, 0, FO.table_scale_of(s.inv_freq), st)
+    if not need_dw:
+        return None
+    if shared is not None:
+        return grads.mark(dev)
+    dw = torch.empty(s.d, device=dev, dtype=torch.bfloat16)
+    _lib.call("spx_rmsnorm_dweight", scratch, scratch.numel() // s.d, s.d, dw, st)
+    return dw
+
+
+def normed_forward(s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next):
+    """``(y, normed, saved)`` as in ``step_forward``."""
+    x2 = _flat(x)
+    nq, h = x2.shape
+    dev = x2.device
+    hq, hkv, d = s.hq, s.hkv, s.d
+    slot_in, slot_o, slot_gu, slot_d = s.slots
+    rstd_in = None
+    if context is not None:
+        c2 = _flat(context)
+        both = torch.cat((c2, _flat(n)))
+        n2 = both[c2.shape[0]:]
+        q_tok, kv_tok = gemm._project(n2, s.wq), gemm._project(both, s.wkv)
+        kv_at = kv_tok.data_ptr()
+    else:
+        rstd_in = torch.empty(nq, device=dev, dtype=torch.float32)
+        both = n2 = _rows(slot_in, nq, h, dev)
+        _lib.call("spx_rmsnorm_fwd", x2, x2.stride(0), gain_in, n2, h, rstd_in, nq, h, s.eps_in, _lib.stream_ptr(dev))
+        q_tok = kv_tok = gemm._project(n2, s.wq)
+        kv_at = kv_tok.data_ptr() + 2 * hq * d
+    nk = both.shape[0]
+    q = torch.empty(1, hq, nq, d, device=dev, dtype=torch.bfloat16)
+    kv = torch.empty(2, 1, hkv, nk, d, device=dev, dtype=torch.bfloat16)
+    rq = _head_norm_rope(q_tok, q_tok.shape[1], q, None, s.q_pos, s, gain_q, s.eps_q, nq, hq, 0)
+    rk = _head_norm_rope(kv_at, kv_tok.shape[1], kv[0], kv[1], s.kv_pos, s, gain_k, s.eps_k, nk, hkv, hkv)
+    att = _rows(slot_o, nq, hq * d, dev)
+    lse = A.masked_forward_into(q, kv[0], kv[1], s.mask, s.scaling, att)
+    y, normed, tail = _tail_forward(s, x2, att, gain_post, gain_next, slot_gu, slot_d, None)
+    return y, normed, (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, *tail)
+
+
+class _NormedLayer(torch.autograd.Function):
+    """``(x, norm(x), context, gains, tokens) -> (y, next norm(y))``, or ``(x, None, None, ...)`` with the input
+    norm in the node."""
+
+    @staticmethod
+    def forward(ctx, s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next, *_tokens):
+        y, normed, saved = normed_forward(s, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next)
+        (_, _, both, n2, _, _, _, _, _, _, att, _, _, _, z, _, act, _) = saved
+        ctx.taken = (s.wq.take(n2), s.wkv.take(both) if s.wkv is not None else -1, s.wo.take(att), s.wgu.take(z),
+                     s.wd.take(act))
+        gains = (gain_in, gain_q, gain_k, gain_post, gain_next)
+        ctx.gain_grads = tuple(getattr(g, "spx_gain_grads", None) for g in gains)
+        ctx.step, ctx.shape, ctx.n_inputs = s, x.shape, 9 + len(_tokens)
+        ctx.context_shape = context.shape if context is not None else None
+        ctx.save_for_backward(*saved, *gains)
+        ctx.set_materialize_grads(False)
+        return y.view(x.shape), normed.view(x.shape)
+
+    @staticmethod
+    def backward(ctx, dy, dn):
+        s = ctx.step
+        if dy is None and dn is None:
+            return (None,) * ctx.n_inputs
+        (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, *tail, gain_in, gain_q, gain_k, gain_post,
+         gain_next) = ctx.saved_tensors
+        needs = ctx.needs_input_grad
+        hq, hkv, d = s.hq, s.hkv, s.d
+        nq, h = n2.shape
+        nk = both.shape[0]
+        dev = n2.device
+        grads_in, grads_q, grads_k, grads_post, grads_next = ctx.gain_grads
+        da, datt, d_post, d_next, tok_o, tok_gu, tok_d = _tail_backward(
+            s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads_next, needs[7:9], ctx.taken[2:])
+        dq, dk, dv = A.masked_backward(q, kv[0], kv[1], att, datt, lse, s.mask, s.scaling)
+        dq_tok = _rows(s.wq.dy_slot(ctx.taken[0], nq), nq, q_tok.shape[1], dev)
+        if s.wkv is not None:
+            dkv_tok = _rows(s.wkv.dy_slot(ctx.taken[1], nk), nk, kv_tok.shape[1], dev)
+            kv_at, dkv_at = kv_tok.data_ptr(), dkv_tok.data_ptr()
+        else:
+            dkv_tok = dq_tok
+            kv_at, dkv_at = kv_tok.data_ptr() + 2 * hq * d, dq_tok.data_ptr() + 2 * hq * d
+        d_gq = _head_norm_rope_backward(q_tok, q_tok.shape[1], dq, None, s.q_pos, s, gain_q, rq, grads_q, needs[5],
+                                        dq_tok, dq_tok.shape[1], nq, hq, 0)
+        d_gk = _head_norm_rope_backward(kv_at, kv_tok.shape[1], dk, dv, s.kv_pos, s, gain_k, rk, grads_k, needs[6],
+                                        dkv_at, dkv_tok.shape[1], nk, hkv, hkv)
+        d_n = gemm._project_back(dq_tok, s.wq)
+        tokens = [s.wq.defer(ctx.taken[0], dq_tok, n2)]
+        d_context = d_in = None
+        if s.wkv is not None:
+            d_both = gemm._project_back(dkv_tok, s.wkv)
+            tokens.append(s.wkv.defer(ctx.taken[1], dkv_tok, both))
+            d_n += d_both[nk - nq:]
+            d_context = d_both[:nk - nq].view(ctx.context_shape) if needs[3] else None
+            dx, d_n = da.view(ctx.shape), d_n.view(ctx.shape)
+        else:
+            dx = _grad_rows(s.grad_slot, nq, h, dev)
+            d_in = FO._norm_backward(grads_in, needs[4], x2, gain_in, d_n, da, rstd_in, dx, nq, h)
+            dx, d_n = dx.view(ctx.shape), None
+        return (None, dx, d_n, d_context, d_in, d_gq, d_gk, d_post, d_next, *tokens, tok_o, tok_gu, tok_d)
+
+
+def _grad_rows(grad_slot, rows: int, cols: int, device):
+    """Where the gradient of a ``gemm.linear_staged`` result goes: the place its weight gradient reads it from,
+    if that has one."""
+    if grad_slot is not None and grad_slot[2] == rows:
+        out = grad_slot[0].dy_slot(grad_slot[1], rows)
+        if out.shape == (rows, cols) and out.is_contiguous():
+            return out
+    return torch.empty(rows, cols, device=device, dtype=torch.bfloat16)
+
+
+def run_normed(s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next):
+    """``(y, normed)``: the layer's output and the next norm of it."""
+    if torch.is_grad_enabled():
+        s.grad_slot = getattr(x, "spx_grad_slot", None)
+        return _NormedLayer.apply(s, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next, *s.tokens())
+    y, normed, _ = normed_forward(s, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next)
+    return y.view(x.shape), normed.view(x.shape)

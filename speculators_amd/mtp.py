@@ -33,6 +33,7 @@ from torch import nn
 from . import attention as A
 from . import fused_ops as FO
 from . import gemm
+from . import layer as LY
 from . import losses as L
 from .eagle3 import MLP, Attention, RMSNorm
 from .hybrid import HybridMTPLayer
@@ -144,6 +145,23 @@ class MTPLayer(nn.Module):
         self.self_attn = Attention(cfg, h, stager)
         self.mlp = MLP(cfg, stager)
 
+    def _step(self, position_ids, inv_freq, mask):
+        """What follows the input projection as one node (``layer.NormedLayer``), or None where it is put together
+        from its parts: no per-head norms, another attention function or head size, a rotary embedding over part
+        of the head, or a graph in which some projection does not train."""
+        att = self.self_attn
+        if not att.qk_norm or not LY.NormedLayer.takes(att, inv_freq, A.ttt_hip_attention_forward):
+            return None
+        W = self._stager.get
+        ws = (W(att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), None, W(att.o_proj.weight),
+              W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight), W(self.mlp.down_proj.weight))
+        if torch.is_grad_enabled() and not all(w is None or w.trainable for w in ws):
+            return None
+        eps = (self.input_layernorm.eps, att.q_norm.eps, att.k_norm.eps, self.post_attention_layernorm.eps,
+               self.final_layernorm.eps)
+        return LY.NormedLayer(*ws, eps, (att.hq, att.hkv, att.d), att.scaling, position_ids, position_ids, inv_freq,
+                              mask)
+
     def forward(self, hidden, embeds, position_ids, inv_freq, mask):
         # both norms write into the halves of the 2H-wide projection input; each residual add is
         # fused into the norm that follows it
@@ -152,6 +170,12 @@ class MTPLayer(nn.Module):
         x = gemm.linear_staged(
             FO.pair_norm_cat(embeds, hidden, self.token_layernorm.gain, self.hidden_layernorm.gain,
                              self.token_layernorm.eps, out=w_in.x_slot(rows)), w_in)
+        step = self._step(position_ids, inv_freq, mask)
+        if step is not None and x.dtype == torch.bfloat16:
+            step.take_slots(rows)
+            att = self.self_attn
+            return LY.run_normed(step, x, None, None, self.input_layernorm.gain, att.q_norm.gain, att.k_norm.gain,
+                                 self.post_attention_layernorm.gain, self.final_layernorm.gain)[1]
         a = self.self_attn(self.input_layernorm(x), position_ids, 0, inv_freq, {}, mask)
         post, final = self.post_attention_layernorm, self.final_layernorm
         w_gu = self._stager.get(self.mlp.gate_proj.weight, self.mlp.up_proj.weight)

@@ -439,3 +439,50 @@ def test_layer_step_node_is_the_layer_from_its_parts(layers, norm_output, fp32, 
     for n, a in want[3].items():
         # (the second layer's q/k/v gradient is one product over the steps instead of one each)
         _close(got[3][n], a.cpu(), rel=1e-2 if layers > 1 else 0.0)
+
+
+@pytest.mark.parametrize("d,t,heads,n_pass", [(64, 1, 1, 0), (64, 77, 3, 3), (128, 1030, 8, 8), (128, 515, 32, 0),
+                                              (256, 33, 2, 2), (256, 4099, 16, 5)])
+def test_head_norm_rope_matches_the_separate_kernels(d, t, heads, n_pass):
+    """The fused per-head norm, rotation and relayout against ``rms_norm`` and ``rope_relayout``: one token, heads that
+    do not divide by the heads per thread, one to four of those; gain sums started and added to."""
+    from speculators_amd import _lib
+    from speculators_amd import fused_ops as FO
+
+    dev = torch.device("cuda:0")
+    torch.manual_seed(d + t)
+    width = (heads + n_pass) * d
+    buf = torch.randn(t, width + 64, device=dev).bfloat16()
+    tok = buf[:, :width]
+    gain = (1 + 0.2 * torch.randn(d, device=dev)).bfloat16()
+    pos = torch.randint(0, 9000, (t,), device=dev)
+    inv_freq = FO.rope_inv_freq(d, 10000.0, dev)
+    st = _lib.stream_ptr(tok.device)
+    out = torch.empty(heads, t, d, device=dev, dtype=torch.bfloat16)
+    passed = torch.full((max(n_pass, 1), t, d), 7.0, device=dev, dtype=torch.bfloat16)
+    rstd = torch.empty(t, heads, device=dev)
+    _lib.call("spx_head_norm_rope", tok, tok.stride(0), out, t * d, passed if n_pass else None, t * d, pos, inv_freq, gain,
+              rstd, t, heads, n_pass, d, 3, 1.0, 1e-6, st)
+    x = tok[:, :heads * d].reshape(t, heads, d).clone().requires_grad_(True)
+    g = gain.clone().requires_grad_(True)
+    want = FO.rope_relayout(FO.rms_norm(x, g, 1e-6).view(1, t, heads * d), pos, inv_freq, heads, True, 3)[0]
+    torch.testing.assert_close(out.float(), want.float(), rtol=1e-2, atol=1e-2)
+    if n_pass:
+        assert torch.equal(passed, tok[:, heads * d:].reshape(t, n_pass, d).transpose(0, 1))
+    dout = torch.randn(heads, t, d, device=dev).bfloat16()
+    dpass = torch.randn(max(n_pass, 1), t, d, device=dev).bfloat16()
+    want.backward(dout)
+    slots = int(_lib.native().spx_rmsnorm_bwd_slots(t * heads, d))
+    parts = torch.empty(slots, d, device=dev)
+    dbuf = torch.full((t, width + 8), 5.0, device=dev, dtype=torch.bfloat16)
+    for acc in (0, 1):
+        _lib.call("spx_head_norm_rope_bwd", tok, tok.stride(0), dout, t * d, dpass if n_pass else None, t * d, pos,
+                  inv_freq, gain, rstd, dbuf, width + 8, parts, acc, t, heads, n_pass, d, 3, 1.0, st)
+        dg = parts.sum(0) / (1 + acc)
+        torch.testing.assert_close(dg, g.grad.float(), rtol=2e-2, atol=2e-2 * float(g.grad.float().abs().max()))
+    torch.testing.assert_close(dbuf[:, :heads * d].reshape(t, heads, d).float(), x.grad.float(), rtol=2e-2, atol=2e-2)
+    if n_pass:
+        assert torch.equal(dbuf[:, heads * d:width].reshape(t, n_pass, d).transpose(0, 1), dpass)
+    assert (dbuf[:, width:] == 5.0).all()
+    _lib.call("spx_head_norm_rope_bwd", tok, tok.stride(0), dout, t * d, dpass if n_pass else None, t * d, pos, inv_freq,
+              gain, rstd, dbuf, width + 8, None, 0, t, heads, n_pass, d, 3, 1.0, st)
