@@ -108,6 +108,24 @@ class _CacheGrads:
     def __init__(self):
         self.task, self.dk, self.dv, self.low = -1, None, None, 0
 
+    def enter(self, n: int):
+        """``(dk, dv)`` to add to for the step with ``n`` steps of keys; ``(None, None)``: its node is the pass's
+        first and makes them."""
+        task = torch._C._current_graph_task_id()
+        if task < 0:
+            raise RuntimeError("the backward of a layer step runs inside a backward pass of autograd only")
+        if self.task != task:
+            self.task, self.dk, self.dv = task, None, None
+            return None, None
+        if n > self.low:
+            raise RuntimeError("the attention node of a later TTT step ran after an earlier step's in one backward pass")
+        return self.dk, self.dv
+
+    def leave(self, n: int, dk, dv):
+        self.low = n
+        # (the first step's node is the last to run: the pass is done with the buffers)
+        self.task, self.dk, self.dv = (self.task, dk, dv) if n > 1 else (-1, None, None)
+
 
 def ttt_forward_into(q, k, v, mask: TTTMask, scaling: float, out) -> torch.Tensor:
     """The forward kernel into ``out`` (``T * Hq * D`` contiguous bf16 elements); returns the row statistics."""
@@ -148,21 +166,6 @@ def _ttt_backward_cached(g: _CacheGrads, q, k, v, out, dout, lse, mask: TTTMask,
     _lib.call(entry, q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo, t, mask.ttt_step,
               hq, hkv, d, scaling, dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1), ws, nbytes,
               _lib.stream_ptr(dev))
-    return dq, dk, dv
-
-
-def ttt_backward_shared(g: _CacheGrads, q, k, v, out, dout, lse, mask: TTTMask, n: int, scaling: float):
-    """``(dq, dk, dv)`` of one step inside a backward pass, dk / dv of the step's OWN keys: complete, because
-    the nodes of all later steps have run."""
-    if torch._C._current_graph_task_id() < 0:
-        raise RuntimeError("the backward of a layer step runs inside a backward pass of autograd only")
-    t = q.shape[2]
-    dq, dk, dv = _ttt_backward_cached(g, q, k, v, out, dout, lse, mask, n, scaling)
-    g.low = n
-    lo = (n - 1) * t
-    dk, dv = dk[:, :, lo:], dv[:, :, lo:]
-    if n == 1:  # the first step's node is the last to run: the pass is done with the buffers
-        g.task, g.dk, g.dv = -1, None, None
     return dq, dk, dv
 
 
@@ -300,7 +303,7 @@ def create_padding_span_mask(attention_mask: torch.Tensor) -> SpanMask:
                     b * n)
 
 
-def _check_span(q, k, v, mask: SpanMask) -> int:
+def _span(q, k, v, mask: SpanMask, scaling: float):
     if q.dim() != 4 or q.shape[0] != 1:
         raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, T, D]")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
@@ -309,11 +312,6 @@ def _check_span(q, k, v, mask: SpanMask) -> int:
     if t != mask.total_seq_len or k.shape[2] != t or v.shape != k.shape:
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match a span mask over "
                          f"{mask.total_seq_len} positions")
-    return t
-
-
-def _span(q, k, v, mask: SpanMask, scaling: float):
-    t = _check_span(q, k, v, mask)
     return _lib.native().attention(q, k, v, mask.row_lo, mask.row_hi, None, None, t, 0, scaling)
 
 
@@ -383,7 +381,7 @@ def create_dflash_mask(document_ids: torch.Tensor, total_seq_len: int,
     return DFlashMask(bounds[0], bounds[1], bounds[2], bounds[3], total_seq_len, n_q)
 
 
-def _check_dflash(q, k, v, mask: DFlashMask) -> int:
+def _dflash(q, k, v, mask: DFlashMask, scaling: float):
     if q.dim() != 4 or q.shape[0] != 1:
         raise ValueError("the packed batch layout has batch size 1: q must be [1, Hq, NQ, D]")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
@@ -392,11 +390,6 @@ def _check_dflash(q, k, v, mask: DFlashMask) -> int:
     if nq != mask.q_len or k.shape[2] != t + nq or v.shape != k.shape:
         raise ValueError(f"q {tuple(q.shape)} / k {tuple(k.shape)} do not match the mask "
                          f"(T {t}, {mask.q_len} block rows)")
-    return t
-
-
-def _dflash(q, k, v, mask: DFlashMask, scaling: float):
-    t = _check_dflash(q, k, v, mask)
     return _lib.native().attention(q, k, v, mask.ctx_lo, mask.ctx_hi, mask.blk_lo, mask.blk_hi, t, 0, scaling)
 
 
@@ -415,57 +408,21 @@ def dflash_hip_attention_forward(module, query, key, value, attention_mask, scal
     return dflash_attention(query, key, value, attention_mask, scaling), None
 
 
-def masked_forward_into(q, k, v, mask, scaling: float, out) -> torch.Tensor:
-    """The forward kernel of any of the masks (a ``TTTMask`` at its first step) into ``out`` (``NQ * Hq * D``
-    contiguous bf16 elements); returns the row statistics."""
+def mask_arguments(mask, nq: int, nk: int) -> tuple:
+    """A mask as the native functions of the layers take it, for ``nq`` query rows and ``nk`` keys."""
     if isinstance(mask, TTTMask):
-        _check_qkv(q, k, v, mask)
-        return ttt_forward_into(q, k, v, mask, scaling, out)
-    t = _check_span(q, k, v, mask) if isinstance(mask, SpanMask) else _check_dflash(q, k, v, mask)
-    _, hq, nq, d = q.shape
-    hkv = k.shape[1]
-    dev = q.device
-    lse = torch.empty(hq, nq, device=dev, dtype=torch.float32)
-    if isinstance(mask, SpanMask):
-        nbytes = _workspace_bytes(nq, hq, hkv, d, False)
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_span_attn_fwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), mask.row_lo, mask.row_hi, nq,
-                  hq, hkv, d, float(scaling), out, lse, ws, nbytes, _lib.stream_ptr(dev))
+        fits, args = nq == mask.total_seq_len and nk == (mask.ttt_step + 1) * nq, (None, None, None)
+        lo, t, step = mask.row_lo, mask.total_seq_len, mask.ttt_step
+    elif isinstance(mask, SpanMask):
+        fits, args = nq == nk == mask.total_seq_len, (mask.row_hi, None, None)
+        lo, t, step = mask.row_lo, nq, 0
     else:
-        nbytes = _lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 0)
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_fwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), mask.ctx_lo, mask.ctx_hi,
-                  mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling), out, lse, ws, nbytes,
-                  _lib.stream_ptr(dev))
-    return lse
-
-
-def masked_backward(q, k, v, out, dout, lse, mask, scaling: float):
-    """``(dq, dk, dv)`` of ``masked_forward_into``."""
-    _, hq, nq, d = q.shape
-    hkv = k.shape[1]
-    dev = q.device
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    st = _lib.stream_ptr(dev)
-    if isinstance(mask, DFlashMask):
-        t = mask.total_seq_len
-        nbytes = _lib.native().spx_dflash_attn_workspace_bytes(t, nq, hq, hkv, d, 1)
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        _lib.call("spx_dflash_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.ctx_lo,
-                  mask.ctx_hi, mask.blk_lo, mask.blk_hi, t, nq, hq, hkv, d, float(scaling), dq, dq.stride(1), dk,
-                  dk.stride(1), dv, dv.stride(1), ws, nbytes, st)
-        return dq, dk, dv
-    nbytes = _workspace_bytes(nq, hq, hkv, d, True)
-    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-    if isinstance(mask, SpanMask):
-        _lib.call("spx_span_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo,
-                  mask.row_hi, nq, hq, hkv, d, float(scaling), dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1),
-                  ws, nbytes, st)
-    else:
-        _lib.call("spx_ttt_attn_bwd", q, q.stride(1), k, k.stride(1), v, v.stride(1), out, dout, lse, mask.row_lo, nq,
-                  mask.ttt_step, hq, hkv, d, float(scaling), dq, dq.stride(1), dk, dk.stride(1), dv, dv.stride(1), ws,
-                  nbytes, st)
-    return dq, dk, dv
+        t, step = mask.total_seq_len, 0
+        fits, args = nq == mask.q_len and nk == t + nq, (mask.ctx_hi, mask.blk_lo, mask.blk_hi)
+        lo = mask.ctx_lo
+    if not fits:
+        raise ValueError(f"{nq} query rows and {nk} keys do not match {type(mask).__name__}")
+    return (lo, *args, t, step)
 
 
 class AttentionRegistry(dict):

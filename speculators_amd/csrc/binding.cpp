@@ -118,13 +118,22 @@ PyObject* set_error(PyObject*, PyObject* cls) {
 }
 
 #define SPX_ROW(fn) {#fn, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&py_##fn)), METH_FASTCALL, nullptr},
+#define SPX_HOST(name, fn) \
+  {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&fn)), METH_FASTCALL, nullptr},
 #define SPX_STATUS(fn) SPX_ROW(fn)
 #define SPX_UNLOCKED(fn) SPX_ROW(fn)
 #define SPX_VALUE(fn) SPX_ROW(fn)
 PyMethodDef g_methods[] = {
 #include "binding_list.h"
-    {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&spx_node_attention)), METH_FASTCALL, nullptr},
-    {"row_loss", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&spx_node_row_loss)), METH_FASTCALL, nullptr},
+    SPX_HOST("attention", spx_node_attention)
+    SPX_HOST("row_loss", spx_node_row_loss)
+    SPX_HOST("product", spx_layer_product)
+    SPX_HOST("tail_forward", spx_layer_tail_forward)
+    SPX_HOST("tail_backward", spx_layer_tail_backward)
+    SPX_HOST("ttt_forward", spx_layer_ttt_forward)
+    SPX_HOST("ttt_backward", spx_layer_ttt_backward)
+    SPX_HOST("normed_forward", spx_layer_normed_forward)
+    SPX_HOST("normed_backward", spx_layer_normed_backward)
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -1,0 +1,299 @@
+// The launches of a decoder layer in sequence: what the Python nodes of layer.py run between their bookkeeping.  A launch
+// out of Python costs 10 us with the tensor it writes, its strides and addresses (2 us for the tensor, 3 to 5 for the
+// call); from here it costs the launch, 3 to 4 us.  Up to a thousand tokens a draft's step was bound by that: 512 tokens of
+// the 1B shape, three TTT steps: 2.50 ms -> 2.36 a pass; three layers of anchored blocks over 1777: 3.76 -> 3.61.
+
+#include "host_common.h"
+
+namespace {
+
+using namespace spx_host;
+
+struct Args {
+  PyObject* const* at;
+  const char* name;
+  Args(const char* fn, PyObject* const* args, Py_ssize_t n, Py_ssize_t want) : at(args), name(fn) {
+    TORCH_CHECK_TYPE(n == want, fn, " takes ", want, " arguments (", n, " given)");
+  }
+  const Tensor& tensor() {
+    const Tensor& t = spx_host::tensor(*at++);
+    need_hip(t);
+    return t;
+  }
+  Tensor maybe() {
+    PyObject* const o = *at++;
+    if (o == Py_None) return Tensor();
+    const Tensor& t = spx_host::tensor(o);
+    need_hip(t);
+    return t;
+  }
+  int64_t integer() {
+    const long long v = PyLong_AsLongLong(*at++);
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+  double number() {
+    const double v = PyFloat_AsDouble(*at++);
+    if (v == -1.0 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+};
+
+PyObject* tuple_of(std::initializer_list<Tensor> ts) {
+  PyObject* const out = PyTuple_New(ts.size());
+  Py_ssize_t i = 0;
+  for (const Tensor& t : ts) PyTuple_SET_ITEM(out, i++, THPVariable_Wrap(t));
+  return out;
+}
+
+const uint16_t* in(const Tensor& t) { return static_cast<const uint16_t*>(t.const_data_ptr()); }
+uint16_t* to(const Tensor& t) { return static_cast<uint16_t*>(t.mutable_data_ptr()); }
+float* floats(const Tensor& t) { return t.defined() ? t.mutable_data_ptr<float>() : nullptr; }
+Tensor rows_or_new(const Tensor& slot, int64_t rows, int64_t cols, const Tensor& like) {
+  return slot.defined() ? slot : at::empty({rows, cols}, like.options().dtype(at::kBFloat16));
+}
+// [.., H] -> [rows, H] with unit inner stride, bf16
+Tensor grad_rows(const Tensor& g) {
+  const Tensor x = g.reshape({-1, g.size(-1)}).to(at::kBFloat16);
+  return x.stride(1) == 1 ? x : x.contiguous();
+}
+
+// How gemm.py routed a product (``Route`` there)
+enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul };
+struct Products {
+  int64_t parts;
+  Tensor ws;  // fp32 partials of products cut along the contraction
+  Tensor operator()(int64_t route, const Tensor& a, const Tensor& b, const Tensor& m_live = Tensor()) const {
+    if (route == kLinear) return at::linear(a, b);
+    if (route == kMatmul) return at::matmul(a, b);
+    const int64_t m = a.size(0), k = a.size(1), n = route == kAutoNN ? b.size(1) : b.size(0);
+    TORCH_CHECK_VALUE(b.size(route == kAutoNN ? 0 : 1) == k, "shape mismatch: a ", a.sizes(), " b ", b.sizes());
+    const Tensor out = at::empty({m, n}, a.options());
+    void* const st = stream_of(a);
+    void* const w = ws.defined() ? ws.mutable_data_ptr() : nullptr;
+    const int64_t wb = ws.defined() ? ws.nbytes() : 0;
+    if (route == kNT)
+      check(spx_gemm_bf16_nt(in(a), a.stride(0), in(b), b.stride(0), to(out), n, m, n, k, st), "spx_gemm_bf16_nt");
+    else if (route == kTail)
+      check(spx_gemm_bf16_nt_tail(in(a), a.stride(0), in(b), b.stride(0), to(out), n, m, n, k, parts, w, wb, st),
+            "spx_gemm_bf16_nt_tail");
+    else
+      check(spx_gemm_bf16_auto(route, in(a), a.stride(0), in(b), b.stride(0), to(out), n, m, n, k,
+                               m_live.defined() ? m_live.const_data_ptr<int32_t>() : nullptr, parts, w, wb, st),
+            "spx_gemm_bf16_auto");
+    return out;
+  }
+};
+
+}  // namespace
+
+// (route, a, b, m_live, parts, workspace) -> a b^T or a b
+PyObject* spx_layer_product(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("product", args, n, 6);
+  const int64_t route = x.integer();
+  const Tensor &a = x.tensor(), &b = x.tensor(), live = x.maybe();
+  const int64_t parts = x.integer();
+  return THPVariable_Wrap(Products{parts, x.maybe()}(route, a, b, live));
+  END_HANDLE_TH_ERRORS
+}
+
+// Behind the attention: o, residual add + norm, gate/up, SwiGLU, down, residual add + the next norm.
+PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("tail_forward", args, n, 17);
+  const Tensor &residual = x.tensor(), &att = x.tensor(), &wo = x.tensor(), &wgu = x.tensor(), &wd = x.tensor(),
+               &gain_post = x.tensor(), &gain_next = x.tensor(), slot_gu = x.maybe(), slot_d = x.maybe(),
+               slot_next = x.maybe();
+  const double eps_post = x.number(), eps_next = x.number();
+  const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
+  const Products product{parts, x.maybe()};
+  const int64_t t = residual.size(0), h = residual.size(1), f = wgu.size(0) / 2;
+  void* const st = stream_of(residual);
+  const Tensor stats = at::empty({2, t}, residual.options().dtype(at::kFloat));
+  float* const rstd = floats(stats);
+  const Tensor o = product(r_o, att, wo);
+  const Tensor mid = at::empty({t, h}, residual.options()), z = rows_or_new(slot_gu, t, h, residual);
+  check(spx_add_rmsnorm_fwd(in(residual), residual.stride(0), in(o), h, to(mid), h, in(gain_post), to(z), h, rstd, t, h,
+                            eps_post, st),
+        "spx_add_rmsnorm_fwd");
+  const Tensor gu = product(r_gu, z, wgu), act = rows_or_new(slot_d, t, f, residual);
+  check(spx_swiglu_rows_fwd(in(gu), 2 * f, in(gu) + f, 2 * f, to(act), f, t, f, st), "spx_swiglu_rows_fwd");
+  const Tensor m = product(r_d, act, wd);
+  const Tensor y = at::empty({t, h}, residual.options()), normed = rows_or_new(slot_next, t, h, residual);
+  check(spx_add_rmsnorm_fwd(in(mid), h, in(m), h, to(y), h, in(gain_next), to(normed), h, rstd + t, t, h, eps_next, st),
+        "spx_add_rmsnorm_fwd");
+  return tuple_of({mid, stats, z, gu, act, y, normed});
+  END_HANDLE_TH_ERRORS
+}
+
+// The way back, from (dy, dn) of (y, normed): -> (gradients of down's, gate/up's and o's outputs, of att).  scratch_*: the
+// partial sums of the gains' gradients (accumulate: added to).
+PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("tail_backward", args, n, 23);
+  const Tensor dy = x.maybe(), dn = x.maybe();
+  const Tensor &mid = x.tensor(), &stats = x.tensor(), &gu = x.tensor(), &y = x.tensor(), &gain_post = x.tensor(),
+               &gain_next = x.tensor(), &bo = x.tensor(), &bgu = x.tensor(), &bd = x.tensor(), slot_d = x.maybe(),
+               slot_gu = x.maybe(), slot_o = x.maybe(), scratch_post = x.maybe();
+  const int64_t acc_post = x.integer();
+  const Tensor scratch_next = x.maybe();
+  const int64_t acc_next = x.integer();
+  const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
+  const Products product{parts, x.maybe()};
+  const int64_t t = y.size(0), h = y.size(1), f = gu.size(1) / 2;
+  void* const st = stream_of(y);
+  const float* const rstd = floats(stats);
+  const Tensor dm = rows_or_new(slot_d, t, h, y);
+  const Tensor dres = dy.defined() ? grad_rows(dy) : Tensor();
+  if (dn.defined()) {
+    const Tensor g = grad_rows(dn);
+    check(spx_rmsnorm_bwd_partial(in(y), h, in(gain_next), in(g), g.stride(0), dres.defined() ? in(dres) : nullptr,
+                                  dres.defined() ? dres.stride(0) : 0, rstd + t, to(dm), h, floats(scratch_next),
+                                  acc_next, t, h, st),
+          "spx_rmsnorm_bwd_partial");
+  } else {
+    dm.copy_(dres);
+  }
+  const Tensor dact = product(r_d, dm, bd), dgu = rows_or_new(slot_gu, t, 2 * f, y);
+  check(spx_swiglu_rows_bwd(in(gu), 2 * f, in(gu) + f, 2 * f, in(dact), f, to(dgu), 2 * f, to(dgu) + f, 2 * f, t, f, st),
+        "spx_swiglu_rows_bwd");
+  const Tensor dz = product(r_gu, dgu, bgu), da = rows_or_new(slot_o, t, h, y);
+  check(spx_rmsnorm_bwd_partial(in(mid), h, in(gain_post), in(dz), h, in(dm), h, rstd, to(da), h, floats(scratch_post),
+                                acc_post, t, h, st),
+        "spx_rmsnorm_bwd_partial");
+  return tuple_of({dm, dgu, da, product(r_o, da, bo)});
+  END_HANDLE_TH_ERRORS
+}
+
+// One TTT step in front of that: q, k, v, rotary embedding, attention over the cache's first (offset + 1) T keys.
+PyObject* spx_layer_ttt_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("ttt_forward", args, n, 18);
+  const Tensor &xin = x.tensor(), &wqkv = x.tensor(), &pos = x.tensor(), &inv_freq = x.tensor(), &k = x.tensor(),
+               &v = x.tensor(), &row_lo = x.tensor(), slot = x.maybe();
+  const int64_t hq = x.integer(), hkv = x.integer(), d = x.integer(), offset = x.integer(), step = x.integer();
+  const double table_scale = x.number(), scaling = x.number();
+  const int64_t route = x.integer(), parts = x.integer();
+  const Products product{parts, x.maybe()};
+  const int64_t t = xin.size(0), at = offset * t * d;
+  TORCH_CHECK_VALUE(k.size(2) >= (offset + 1) * t && row_lo.numel() == t && pos.numel() == t && step == offset,
+                    "the layer's cache, mask and positions do not fit step ", offset, " of ", t, " tokens");
+  void* const st = stream_of(xin);
+  const Tensor qkv = product(route, xin, wqkv);
+  const Tensor q = at::empty({1, hq, t, d}, xin.options());
+  check(spx_rope_qkv(to(qkv), qkv.size(1), to(q), t * d, to(k) + at, k.stride(1), to(v) + at, v.stride(1),
+                     pos.const_data_ptr<int64_t>(), inv_freq.const_data_ptr<float>(), t, hq, hkv, d,
+                     2 * inv_freq.numel(), 0, offset, table_scale, st),
+        "spx_rope_qkv");
+  const Tensor att = rows_or_new(slot, t, hq * d, xin);
+  const Tensor lse = attention_forward(q, k, v, Mask{row_lo, {}, {}, {}, t, step}, scaling, att);
+  return tuple_of({q, att, lse});
+  END_HANDLE_TH_ERRORS
+}
+
+// -> (gradient of q, k, v's product, of its input, dk, dv of all keys up to this step).  dk, dv None: this step's node is
+// the first of the pass and makes them; otherwise they are added to.
+PyObject* spx_layer_ttt_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("ttt_backward", args, n, 21);
+  const Tensor &q = x.tensor(), &k = x.tensor(), &v = x.tensor(), &att = x.tensor(), &datt = x.tensor(),
+               &lse = x.tensor(), &row_lo = x.tensor();
+  Tensor dk = x.maybe(), dv = x.maybe();
+  const Tensor slot = x.maybe();
+  const Tensor &pos = x.tensor(), &inv_freq = x.tensor();
+  const int64_t offset = x.integer();
+  const double table_scale = x.number(), scaling = x.number();
+  const Tensor& w = x.tensor();
+  const int64_t n_qkv = x.integer(), route = x.integer(), parts = x.integer();
+  const Products product{parts, x.maybe()};
+  const int64_t step = x.integer();
+  const int64_t hq = q.size(1), t = q.size(2), d = q.size(3), hkv = k.size(1), keys = (offset + 1) * t, at = offset * t * d;
+  void* const st = stream_of(q);
+  const bool add = dk.defined();
+  if (!add) {
+    dk = at::empty({1, hkv, keys, d}, q.options());
+    dv = at::empty({1, hkv, keys, d}, q.options());
+  }
+  TORCH_CHECK_VALUE(dk.size(2) >= keys && dv.size(2) >= keys && k.size(2) >= keys, "gradients of ", keys, " keys");
+  const Tensor dq = at::empty_like(q);
+  const int64_t nb = spx_ttt_attn_workspace_bytes(t, hq, hkv, d, 1);
+  const Tensor ws = bytes(nb, q);
+  check((add ? spx_ttt_attn_bwd_accumulate : spx_ttt_attn_bwd)(
+            in(q), q.stride(1), in(k), k.stride(1), in(v), v.stride(1), in(att), in(datt), lse.const_data_ptr<float>(),
+            row_lo.const_data_ptr<int32_t>(), t, step, hq, hkv, d, scaling, to(dq), dq.stride(1), to(dk), dk.stride(1),
+            to(dv), dv.stride(1), ws.mutable_data_ptr(), nb, st),
+        "spx_ttt_attn_bwd");
+  const Tensor dqkv = rows_or_new(slot, t, n_qkv, q);
+  check(spx_rope_qkv(to(dqkv), n_qkv, to(dq), dq.stride(1), to(dk) + at, dk.stride(1), to(dv) + at, dv.stride(1),
+                     pos.const_data_ptr<int64_t>(), inv_freq.const_data_ptr<float>(), t, hq, hkv, d,
+                     2 * inv_freq.numel(), 1, offset, table_scale, st),
+        "spx_rope_qkv");
+  return tuple_of({dqkv, product(route, dqkv, w), dk, dv});
+  END_HANDLE_TH_ERRORS
+}
+
+// Per-head norms, rotation and attention of a layer whose q rows are the last of its key rows or all of them.  kv_column:
+// where k begins in a row of kv_tok (v behind it).
+PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("normed_forward", args, n, 22);
+  const Tensor &q_tok = x.tensor(), &kv_tok = x.tensor(), &q_pos = x.tensor(), &kv_pos = x.tensor(),
+               &inv_freq = x.tensor(), &gain_q = x.tensor(), &gain_k = x.tensor(), slot = x.maybe();
+  const int64_t kv_column = x.integer(), hq = x.integer(), hkv = x.integer(), d = x.integer();
+  const double table_scale = x.number(), scaling = x.number(), eps_q = x.number(), eps_k = x.number();
+  const Tensor &lo = x.tensor(), hi = x.maybe(), blo = x.maybe(), bhi = x.maybe();
+  const int64_t T = x.integer(), step = x.integer();
+  const int64_t nq = q_tok.size(0), nk = kv_tok.size(0);
+  TORCH_CHECK_VALUE(q_pos.numel() == nq && kv_pos.numel() == nk, "positions of ", nq, " and ", nk, " rows");
+  void* const st = stream_of(q_tok);
+  const Tensor q = at::empty({1, hq, nq, d}, q_tok.options()), kv = at::empty({2, 1, hkv, nk, d}, q_tok.options()),
+               rq = at::empty({nq, hq}, q_tok.options().dtype(at::kFloat)),
+               rk = at::empty({nk, hkv}, q_tok.options().dtype(at::kFloat));
+  const Tensor k = kv.select(0, 0), v = kv.select(0, 1);
+  const float* const f = inv_freq.const_data_ptr<float>();
+  check(spx_head_norm_rope(in(q_tok), q_tok.stride(0), to(q), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(), f,
+                           in(gain_q), floats(rq), nq, hq, 0, d, 0, table_scale, eps_q, st),
+        "spx_head_norm_rope");
+  check(spx_head_norm_rope(in(kv_tok) + kv_column, kv_tok.stride(0), to(k), nk * d, to(v), nk * d,
+                           kv_pos.const_data_ptr<int64_t>(), f, in(gain_k), floats(rk), nk, hkv, hkv, d, 0, table_scale,
+                           eps_k, st),
+        "spx_head_norm_rope");
+  const Tensor att = rows_or_new(slot, nq, hq * d, q_tok);
+  const Tensor lse = attention_forward(q, k, v, Mask{lo, hi, blo, bhi, T, step}, scaling, att);
+  return tuple_of({q, kv, rq, rk, att, lse});
+  END_HANDLE_TH_ERRORS
+}
+
+// -> (gradients of the two products).  Without separate k, v (kv_column > 0) both are one.
+PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("normed_backward", args, n, 29);
+  const Tensor &q_tok = x.tensor(), &kv_tok = x.tensor(), &q = x.tensor(), &kv = x.tensor(), &rq = x.tensor(),
+               &rk = x.tensor(), &att = x.tensor(), &datt = x.tensor(), &lse = x.tensor(), &q_pos = x.tensor(),
+               &kv_pos = x.tensor(), &inv_freq = x.tensor(), &gain_q = x.tensor(), &gain_k = x.tensor(),
+               slot_q = x.maybe(), slot_kv = x.maybe(), scratch_q = x.maybe();
+  const int64_t acc_q = x.integer();
+  const Tensor scratch_k = x.maybe();
+  const int64_t acc_k = x.integer(), kv_column = x.integer();
+  const double table_scale = x.number(), scaling = x.number();
+  const Tensor &lo = x.tensor(), hi = x.maybe(), blo = x.maybe(), bhi = x.maybe();
+  const int64_t T = x.integer(), step = x.integer();
+  const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = kv.size(2), nk = kv.size(3);
+  void* const st = stream_of(q);
+  const auto [dq, dk, dv] = attention_backward(q, kv.select(0, 0), kv.select(0, 1), att, datt, lse,
+                                               Mask{lo, hi, blo, bhi, T, step}, scaling);
+  const Tensor dq_tok = rows_or_new(slot_q, nq, q_tok.size(1), q),
+               dkv_tok = kv_column ? dq_tok : rows_or_new(slot_kv, nk, kv_tok.size(1), q);
+  const float* const f = inv_freq.const_data_ptr<float>();
+  check(spx_head_norm_rope_bwd(in(q_tok), q_tok.stride(0), in(dq), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(),
+                               f, in(gain_q), floats(rq), to(dq_tok), dq_tok.stride(0), floats(scratch_q), acc_q, nq, hq,
+                               0, d, 0, table_scale, st),
+        "spx_head_norm_rope_bwd");
+  check(spx_head_norm_rope_bwd(in(kv_tok) + kv_column, kv_tok.stride(0), in(dk), nk * d, in(dv), nk * d,
+                               kv_pos.const_data_ptr<int64_t>(), f, in(gain_k), floats(rk), to(dkv_tok) + kv_column,
+                               dkv_tok.stride(0), floats(scratch_k), acc_k, nk, hkv, hkv, d, 0, table_scale, st),
+        "spx_head_norm_rope_bwd");
+  return tuple_of({dq_tok, dkv_tok});
+  END_HANDLE_TH_ERRORS
+}

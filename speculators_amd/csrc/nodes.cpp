@@ -3,75 +3,94 @@
 // (argument and context objects, the interpreter's lock taken again on the engine's thread); these cost 5.
 // 1024 tokens of the 1B attention shape, forward and backward issued: 150 -> 75 us; a loss function 130 -> 75 us.
 
-#include <Python.h>
-
-#include <c10/hip/HIPStream.h>
-#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
-#include <torch/csrc/autograd/python_variable.h>
 
-#include "../../include/spx.h"
-#include "nodes.h"
+#include "host_common.h"
+
+namespace spx_host {
+
+static const int32_t* i32(const Tensor& t) { return static_cast<const int32_t*>(t.const_data_ptr()); }
+
+Tensor attention_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Mask& m, double scaling,
+                         const Tensor& out) {
+  const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = k.size(1);
+  const Tensor lse = at::empty({hq, nq}, q.options().dtype(at::kFloat));
+  const bool blocks = m.blo.defined();
+  const int64_t n = blocks ? spx_dflash_attn_workspace_bytes(m.T, nq, hq, hkv, d, 0)
+                           : spx_ttt_attn_workspace_bytes(nq, hq, hkv, d, 0);
+  const Tensor ws = bytes(n, q);
+  void* const st = stream_of(q);
+  float* const l = lse.mutable_data_ptr<float>();
+  if (blocks)
+    check(spx_dflash_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                              v.stride(1), i32(m.lo), i32(m.hi), i32(m.blo), i32(m.bhi), m.T, nq, hq, hkv, d, scaling,
+                              out.mutable_data_ptr(), l, ws.mutable_data_ptr(), n, st),
+          "spx_dflash_attn_fwd");
+  else if (m.hi.defined())
+    check(spx_span_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                            v.stride(1), i32(m.lo), i32(m.hi), nq, hq, hkv, d, scaling, out.mutable_data_ptr(), l,
+                            ws.mutable_data_ptr(), n, st),
+          "spx_span_attn_fwd");
+  else
+    check(spx_ttt_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                           v.stride(1), i32(m.lo), nq, m.step, hq, hkv, d, scaling, out.mutable_data_ptr(), l,
+                           ws.mutable_data_ptr(), n, st),
+          "spx_ttt_attn_fwd");
+  return lse;
+}
+
+std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& q, const Tensor& k, const Tensor& v,
+                                                      const Tensor& out, const Tensor& dout, const Tensor& lse,
+                                                      const Mask& m, double scaling) {
+  const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = k.size(1);
+  const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+  const bool blocks = m.blo.defined();
+  const int64_t n = blocks ? spx_dflash_attn_workspace_bytes(m.T, nq, hq, hkv, d, 1)
+                           : spx_ttt_attn_workspace_bytes(nq, hq, hkv, d, 1);
+  const Tensor ws = bytes(n, q);
+  void* const st = stream_of(q);
+  const float* const l = lse.const_data_ptr<float>();
+  if (blocks)
+    check(spx_dflash_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                              v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), l, i32(m.lo), i32(m.hi),
+                              i32(m.blo), i32(m.bhi), m.T, nq, hq, hkv, d, scaling, dq.mutable_data_ptr(), dq.stride(1),
+                              dk.mutable_data_ptr(), dk.stride(1), dv.mutable_data_ptr(), dv.stride(1),
+                              ws.mutable_data_ptr(), n, st),
+          "spx_dflash_attn_bwd");
+  else if (m.hi.defined())
+    check(spx_span_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                            v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), l, i32(m.lo), i32(m.hi), nq, hq,
+                            hkv, d, scaling, dq.mutable_data_ptr(), dq.stride(1), dk.mutable_data_ptr(), dk.stride(1),
+                            dv.mutable_data_ptr(), dv.stride(1), ws.mutable_data_ptr(), n, st),
+          "spx_span_attn_bwd");
+  else
+    check(spx_ttt_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
+                           v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), l, i32(m.lo), nq, m.step, hq, hkv,
+                           d, scaling, dq.mutable_data_ptr(), dq.stride(1), dk.mutable_data_ptr(), dk.stride(1),
+                           dv.mutable_data_ptr(), dv.stride(1), ws.mutable_data_ptr(), n, st),
+          "spx_ttt_attn_bwd");
+  return {dq, dk, dv};
+}
+
+}  // namespace spx_host
 
 namespace {
 
-using at::Tensor;
+using namespace spx_host;
 using torch::autograd::AutogradContext;
 using torch::autograd::Function;
 using torch::autograd::variable_list;
 
-void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
-
-// The error goes through the autograd engine as the Python exception it is.
-[[noreturn]] void fail(const char* fmt, const char* a, long rc = 0, const char* b = "") {
-  PyGILState_STATE g = PyGILState_Ensure();
-  PyErr_Format(spx_error_class(), fmt, a, rc, b);
-  python_error e;
-  e.persist();
-  PyGILState_Release(g);
-  throw e;
-}
-void check(int rc, const char* name) {
-  if (rc != 0) fail("%s failed (%ld): %s", name, rc, spx_last_error());
-}
-void need_hip(const Tensor& t) {
-  if (!t.is_cuda()) fail("%s", "libspx_hip works on HIP device tensors only (got a CPU tensor)");
-}
-Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n}, like.options().dtype(at::kByte)); }
-
 // ---------------------------------------------------------------- attention
-// lo only: TTT (step, T keys per step); lo, hi: one interval per row; blo, bhi too: anchored blocks behind T context keys
 struct Attention : Function<Attention> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& lo,
                         const std::optional<Tensor>& hi_, const std::optional<Tensor>& blo_,
                         const std::optional<Tensor>& bhi_, int64_t T, int64_t step, double scaling) {
-    const Tensor hi = hi_.value_or(Tensor()), blo = blo_.value_or(Tensor()), bhi = bhi_.value_or(Tensor());
+    const Mask m{lo, hi_.value_or(Tensor()), blo_.value_or(Tensor()), bhi_.value_or(Tensor()), T, step};
     const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous();
-    const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = k.size(1);
-    const Tensor out = at::empty({1, nq, hq, d}, q.options());
-    const Tensor lse = at::empty({hq, nq}, q.options().dtype(at::kFloat));
-    const bool blocks = blo.defined(), span = hi.defined();
-    const int64_t n = blocks ? spx_dflash_attn_workspace_bytes(T, nq, hq, hkv, d, 0)
-                             : spx_ttt_attn_workspace_bytes(nq, hq, hkv, d, 0);
-    const Tensor ws = bytes(n, q);
-    void* const st = stream_of(q);
-    auto i32 = [](const Tensor& t) { return static_cast<const int32_t*>(t.const_data_ptr()); };
-    if (blocks)
-      check(spx_dflash_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                                v.stride(1), i32(lo), i32(hi), i32(blo), i32(bhi), T, nq, hq, hkv, d, scaling,
-                                out.mutable_data_ptr(), lse.mutable_data_ptr<float>(), ws.mutable_data_ptr(), n, st),
-            "spx_dflash_attn_fwd");
-    else if (span)
-      check(spx_span_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                              v.stride(1), i32(lo), i32(hi), nq, hq, hkv, d, scaling, out.mutable_data_ptr(),
-                              lse.mutable_data_ptr<float>(), ws.mutable_data_ptr(), n, st),
-            "spx_span_attn_fwd");
-    else
-      check(spx_ttt_attn_fwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                             v.stride(1), i32(lo), nq, step, hq, hkv, d, scaling, out.mutable_data_ptr(),
-                             lse.mutable_data_ptr<float>(), ws.mutable_data_ptr(), n, st),
-            "spx_ttt_attn_fwd");
-    ctx->save_for_backward({q, k, v, out, lse, lo, hi, blo, bhi});
+    const Tensor out = at::empty({1, q.size(2), q.size(1), q.size(3)}, q.options());
+    const Tensor lse = attention_forward(q, k, v, m, scaling, out);
+    ctx->save_for_backward({q, k, v, out, lse, m.lo, m.hi, m.blo, m.bhi});
     ctx->saved_data["T"] = T;
     ctx->saved_data["step"] = step;
     ctx->saved_data["scaling"] = scaling;
@@ -80,39 +99,9 @@ struct Attention : Function<Attention> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
-    const Tensor &q = s[0], &k = s[1], &v = s[2], &out = s[3], &lse = s[4], &lo = s[5], &hi = s[6], &blo = s[7], &bhi = s[8];
-    const int64_t T = ctx->saved_data["T"].toInt(), step = ctx->saved_data["step"].toInt();
-    const double scaling = ctx->saved_data["scaling"].toDouble();
-    const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = k.size(1);
-    const Tensor dout = grads[0].to(at::kBFloat16).contiguous();
-    const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    const bool blocks = blo.defined(), span = hi.defined();
-    const int64_t n = blocks ? spx_dflash_attn_workspace_bytes(T, nq, hq, hkv, d, 1)
-                             : spx_ttt_attn_workspace_bytes(nq, hq, hkv, d, 1);
-    const Tensor ws = bytes(n, q);
-    void* const st = stream_of(q);
-    auto i32 = [](const Tensor& t) { return static_cast<const int32_t*>(t.const_data_ptr()); };
-    if (blocks)
-      check(spx_dflash_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                                v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), lse.const_data_ptr<float>(),
-                                i32(lo), i32(hi), i32(blo), i32(bhi), T, nq, hq, hkv, d, scaling, dq.mutable_data_ptr(),
-                                dq.stride(1), dk.mutable_data_ptr(), dk.stride(1), dv.mutable_data_ptr(), dv.stride(1),
-                                ws.mutable_data_ptr(), n, st),
-            "spx_dflash_attn_bwd");
-    else if (span)
-      check(spx_span_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                              v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), lse.const_data_ptr<float>(),
-                              i32(lo), i32(hi), nq, hq, hkv, d, scaling, dq.mutable_data_ptr(), dq.stride(1),
-                              dk.mutable_data_ptr(), dk.stride(1), dv.mutable_data_ptr(), dv.stride(1),
-                              ws.mutable_data_ptr(), n, st),
-            "spx_span_attn_bwd");
-    else
-      check(spx_ttt_attn_bwd(q.const_data_ptr(), q.stride(1), k.const_data_ptr(), k.stride(1), v.const_data_ptr(),
-                             v.stride(1), out.const_data_ptr(), dout.const_data_ptr(), lse.const_data_ptr<float>(),
-                             i32(lo), nq, step, hq, hkv, d, scaling, dq.mutable_data_ptr(), dq.stride(1),
-                             dk.mutable_data_ptr(), dk.stride(1), dv.mutable_data_ptr(), dv.stride(1),
-                             ws.mutable_data_ptr(), n, st),
-            "spx_ttt_attn_bwd");
+    const Mask m{s[5], s[6], s[7], s[8], ctx->saved_data["T"].toInt(), ctx->saved_data["step"].toInt()};
+    const auto [dq, dk, dv] = attention_backward(s[0], s[1], s[2], s[3], grads[0].to(at::kBFloat16).contiguous(), s[4],
+                                                 m, ctx->saved_data["scaling"].toDouble());
     return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -161,15 +150,6 @@ struct RowLoss : Function<RowLoss> {
     return {grad.view(shape), Tensor(), Tensor()};
   }
 };
-
-const Tensor& tensor(PyObject* o) {
-  TORCH_CHECK_TYPE(THPVariable_Check(o), "expected a tensor, got ", Py_TYPE(o)->tp_name);
-  return THPVariable_Unpack(o);
-}
-std::optional<Tensor> tensor_or_none(PyObject* o) {
-  if (o == Py_None) return std::nullopt;
-  return tensor(o);
-}
 
 }  // namespace
 

@@ -7,3 +7,12 @@ PyObject* spx_error_class();  // SpxError
 PyObject* spx_node_attention(PyObject*, PyObject* const* args, Py_ssize_t n);
 // row_loss(op, logits [..., V], targets) -> float32 [...]
 PyObject* spx_node_row_loss(PyObject*, PyObject* const* args, Py_ssize_t n);
+
+// The launches of a decoder layer in sequence (layer_host.cpp), called by layer.py; arguments positional, as read there.
+PyObject* spx_layer_product(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_ttt_forward(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_ttt_backward(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t n);

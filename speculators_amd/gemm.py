@@ -112,14 +112,14 @@ def _plan(form: int, m: int, n: int, k: int, parts: int):
             lib.spx_gemm_auto_us(form, m, n, k, parts))
 
 
-def _auto(form: int, a, b, out, m: int, n: int, k: int, ws_numel: int, m_live=None):
-    if out is None:
-        out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
+# how a product runs, as csrc/layer_host.cpp numbers it: on spx_gemm_bf16_auto (NT or NN form), on the 256 x 256 kernel
+# without or with its last round cut, or in the library
+AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL = range(6)
+
+
+def _auto(form: int, a, b, ws_numel: int, m_live=None):
     ws = _split_workspace(a.device, ws_numel) if ws_numel else None
-    _lib.call("spx_gemm_bf16_auto", form, a, a.stride(0), b, b.stride(0), out,
-              out.stride(0), m, n, k, m_live, TAIL_PARTS, ws, ws_numel * 4,
-              _lib.stream_ptr(a.device))
-    return out
+    return _lib.native().product(form, a, b, m_live, TAIL_PARTS, ws)
 
 
 def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = None) -> torch.Tensor:
@@ -133,7 +133,7 @@ def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = No
     if k == b.shape[1] and k % 8 == 0 and a.stride(1) == 1 and b.stride(1) == 1 and a.dtype == b.dtype == torch.bfloat16:
         big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
         if not big:
-            return _auto(0, a, b, None, m, n, k, ws_numel, m_live)
+            return _auto(AUTO_NT, a, b, ws_numel, m_live)
     return gemm_nt(a, b, m_live=m_live, split=m_live is not None)
 
 
@@ -151,7 +151,7 @@ def matmul_nn(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     lies, no transposed copy of it."""
     m, k = a.shape
     n = b.shape[1]
-    return _auto(1, a, b, None, m, n, k, _plan(1, m, n, k, TAIL_PARTS)[1])
+    return _auto(AUTO_NN, a, b, _plan(1, m, n, k, TAIL_PARTS)[1])
 
 
 # microseconds to transpose a million weight elements (spx_transpose_bf16: 4 bytes each at 3.8 TB/s)
@@ -349,6 +349,52 @@ def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
     if DECODER_GEMM != "hipblaslt" and dy2.shape[1] % 8 == 0 and dy2.stride(0) % 8 == 0 and dy2.stride(1) == 1:
         return input_gradient(dy2, staged)
     return torch.matmul(dy2, staged.w)
+
+
+@functools.lru_cache(maxsize=4096)
+def _forward_route(mode: str, parts: int, m: int, n: int, k: int):
+    """``(route, workspace elements)`` of ``_project`` for contiguous rows."""
+    if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k)):
+        return LINEAR, 0
+    big, ws_numel, _ = _plan(0, m, n, k, parts)
+    if not big and k % 8 == 0:
+        return AUTO_NT, ws_numel
+    rem = (-(-m // 256) * -(-n // 256)) % _CUS
+    if parts > 1 and 0 < rem <= _CUS // 2 and k >= 64 * 16 * 2:
+        return TAIL, _lib.native().spx_gemm_tail_workspace_bytes() // 4
+    return NT, 0
+
+
+def forward_route(m: int, staged):
+    return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *staged.w.shape)
+
+
+@functools.lru_cache(maxsize=4096)
+def _backward_route(mode: str, parts: int, m: int, k: int, n: int, ld: int, aligned: bool, copy_us: float):
+    """``(route, workspace elements, on the transposed copy)`` of ``_project_back`` for contiguous rows."""
+    if mode == "hipblaslt" or k % 8:
+        return MATMUL, 0, False
+    if aligned and n % 8 == 0 and ld % 8 == 0 and (k + 256) * ld * 2 < _MAX_SPAN and 257 * k * 2 < _MAX_SPAN:
+        _, ws_numel, us = _plan(1, m, n, k, parts)
+        if us <= _plan(0, m, n, k, parts)[2] + copy_us:
+            return AUTO_NN, ws_numel, False
+    return (*_forward_route("spx", parts, m, n, k), True)
+
+
+def backward_route(m: int, staged):
+    """``(route, workspace elements, right operand)`` of the input gradient of a product with ``m`` rows."""
+    w = staged.w
+    k, n = w.shape
+    copy_us = 0.0 if staged.has_wt or not staged.trainable else (3.0 + _TRANSPOSE_US * 1e-6 * k * n) / staged.uses
+    route, ws, transposed = _backward_route(DECODER_GEMM, TAIL_PARTS, m, k, n, w.stride(0), w.data_ptr() % 16 == 0,
+                                            copy_us)
+    return route, ws, staged.wt if transposed else w
+
+
+def workspace_for(device, *numels):
+    """The workspace for products that ask for that many elements (one stream: they run one after the other)."""
+    n = max(numels)
+    return _split_workspace(device, n) if n else None
 
 
 class _StagedLinear(torch.autograd.Function):

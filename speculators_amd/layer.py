@@ -63,14 +63,11 @@ def step_forward(s: LayerStep, a, b, gain_a, gain_b, gain_post, gain_next):
         residual = b2
     else:  # a: the residual stream, b: its norm
         rstd_in, xin, residual = None, b2, a2
-    hq, hkv, d = s.hq, s.hkv, s.d
-    qkv = gemm._project(xin, s.wqkv)
-    scale = FO.table_scale_of(s.inv_freq)
-    q, _, _ = gemm._qkv_heads(qkv, s.positions, s.inv_freq, hq, hkv, d, s.offset, scale, s.cache.window(s.offset))
-    n = (s.offset + 1) * t
-    k, v = s.cache.k[:, :, :n], s.cache.v[:, :, :n]
-    att = _rows(slot_o, t, hq * d, dev)
-    lse = A.ttt_forward_into(q, k, v, s.mask, s.scaling, att)
+    cache, mask = s.cache, s.mask
+    route, ws = gemm.forward_route(t, s.wqkv)
+    q, att, lse = _lib.native().ttt_forward(
+        xin, s.wqkv.w, s.positions, s.inv_freq, cache.k, cache.v, mask.row_lo, slot_o, s.hq, s.hkv, s.d, s.offset,
+        mask.ttt_step, FO.table_scale_of(s.inv_freq), s.scaling, route, gemm.TAIL_PARTS, gemm.workspace_for(dev, ws))
     y, normed, tail = _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_next)
     return y, normed, (a2, b2, rstd_in, xin, q, att, lse, *tail)
 
@@ -78,25 +75,41 @@ def step_forward(s: LayerStep, a, b, gain_a, gain_b, gain_post, gain_next):
 def _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_next):
     """What follows the attention: output projection, residual add and norm, MLP, residual add and the norm
     that reads the layer's output."""
-    t, h = residual.shape
-    dev = residual.device
-    st = _lib.stream_ptr(dev)
-    o = gemm._project(att, s.wo)
-    stats = torch.empty(2, t, device=dev, dtype=torch.float32)
-    mid = torch.empty(t, h, device=dev, dtype=torch.bfloat16)
-    z = _rows(slot_gu, t, h, dev)
-    _lib.call("spx_add_rmsnorm_fwd", residual, residual.stride(0), o, h, mid, h, gain_post, z, h, stats, t, h,
-              s.eps_post, st)
-    gu = gemm._project(z, s.wgu)
-    f = gu.shape[1] // 2
-    act = _rows(slot_d, t, f, dev)
-    base = gu.data_ptr()
-    _lib.call("spx_swiglu_rows_fwd", base, 2 * f, base + 2 * f, 2 * f, act, f, t, f, st)
-    m = gemm._project(act, s.wd)
-    y = torch.empty(t, h, device=dev, dtype=torch.bfloat16)
-    normed = _rows(slot_next, t, h, dev)
-    _lib.call("spx_add_rmsnorm_fwd", mid, h, m, h, y, h, gain_next, normed, h, stats[1], t, h, s.eps_next, st)
-    return y, normed, (mid, stats, z, gu, act, y)
+    t = residual.shape[0]
+    routes, sizes = zip(*(gemm.forward_route(t, w) for w in (s.wo, s.wgu, s.wd)))
+    *tail, y, normed = _lib.native().tail_forward(
+        residual, att, s.wo.w, s.wgu.w, s.wd.w, gain_post, gain_next, slot_gu, slot_d, slot_next, s.eps_post, s.eps_next,
+        *routes, gemm.TAIL_PARTS, gemm.workspace_for(residual.device, *sizes))
+    return y, normed, (*tail, y)
+
+
+class _GainSum:
+    """Where one use of a gain leaves the partial sums of its gradient, and what its node returns for it."""
+
+    __slots__ = ("grads", "scratch", "acc", "own")
+
+    def __init__(self, grads, needed: bool, rows: int, h: int, device):
+        self.grads, self.scratch, self.acc, self.own = grads, None, 0, False
+        if not needed:
+            self.grads = None
+            return
+        shared = grads.target(rows, h, device) if grads is not None else None
+        if shared is not None:
+            self.scratch, self.acc = shared
+        else:
+            slots = int(_lib.native().spx_rmsnorm_bwd_slots(rows, h))
+            self.scratch, self.own = torch.empty(slots, h, device=device, dtype=torch.float32), True
+
+    def result(self):
+        if self.scratch is None:
+            return None
+        dev = self.scratch.device
+        if not self.own:
+            return self.grads.mark(dev)
+        slots, h = self.scratch.shape
+        dw = torch.empty(h, device=dev, dtype=torch.bfloat16)
+        _lib.call("spx_rmsnorm_dweight", self.scratch, slots, h, dw, _lib.stream_ptr(dev))
+        return dw
 
 
 def _tail_backward(s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads_next, needs, taken):
@@ -105,31 +118,16 @@ def _tail_backward(s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads
     mid, stats, z, gu, act, y = tail
     slot_o, slot_gu, slot_d = taken
     t, h = y.shape
-    f = act.shape[1]
     dev = y.device
-    st = _lib.stream_ptr(dev)
-    if dy is not None:
-        dy = _flat(dy).to(torch.bfloat16)
-    dm = _rows(s.wd.dy_slot(slot_d, t), t, h, dev)
-    d_next = None
-    if dn is not None:
-        d_next = FO._norm_backward(grads_next, needs[1], y, gain_next, _flat(dn).to(torch.bfloat16), dy, stats[1],
-                                   dm, t, h)
-    else:
-        dm.copy_(dy)
-    dact = gemm._project_back(dm, s.wd)
-    tok_d = s.wd.defer(slot_d, dm, act)
-    dgu = _rows(s.wgu.dy_slot(slot_gu, t), t, 2 * f, dev)
-    base, dbase = gu.data_ptr(), dgu.data_ptr()
-    _lib.call("spx_swiglu_rows_bwd", base, 2 * f, base + 2 * f, 2 * f, dact, f, dbase, 2 * f, dbase + 2 * f, 2 * f,
-              t, f, st)
-    dz = gemm._project_back(dgu, s.wgu)
-    tok_gu = s.wgu.defer(slot_gu, dgu, z)
-    da = _rows(s.wo.dy_slot(slot_o, t), t, h, dev)
-    d_post = FO._norm_backward(grads_post, needs[0], mid, gain_post, dz, dm, stats[0], da, t, h)
-    datt = gemm._project_back(da, s.wo)
-    tok_o = s.wo.defer(slot_o, da, att)
-    return da, datt, d_post, d_next, tok_o, tok_gu, tok_d
+    nxt = _GainSum(grads_next, needs[1] and dn is not None, t, h, dev)
+    post = _GainSum(grads_post, needs[0], t, h, dev)
+    routes, sizes, right = zip(*(gemm.backward_route(t, w) for w in (s.wo, s.wgu, s.wd)))
+    dm, dgu, da, datt = _lib.native().tail_backward(
+        dy, dn, mid, stats, gu, y, gain_post, gain_next, *right, s.wd.dy_slot(slot_d, t), s.wgu.dy_slot(slot_gu, t),
+        s.wo.dy_slot(slot_o, t), post.scratch, post.acc, nxt.scratch, nxt.acc, *routes, gemm.TAIL_PARTS,
+        gemm.workspace_for(dev, *sizes))
+    tok_d, tok_gu, tok_o = s.wd.defer(slot_d, dm, act), s.wgu.defer(slot_gu, dgu, z), s.wo.defer(slot_o, da, att)
+    return da, datt, post.result(), nxt.result(), tok_o, tok_gu, tok_d
 
 
 class _LayerStep(torch.autograd.Function):
@@ -160,19 +158,19 @@ class _LayerStep(torch.autograd.Function):
         s = ctx.step
         needs = ctx.needs_input_grad
         t = y.shape[0]
-        dev = y.device
         slot_qkv = ctx.taken[0]
         grads_a, grads_b, grads_post, grads_next = ctx.gain_grads
         da, datt, d_post, d_next, tok_o, tok_gu, tok_d = _tail_backward(
             s, dy, dn, att, (mid, stats, z, gu, act, y), gain_post, gain_next, grads_post, grads_next, needs[5:7],
             ctx.taken[1:])
-        step_no = s.offset + 1
-        k, v = s.cache.k[:, :, :step_no * t], s.cache.v[:, :, :step_no * t]
-        dq, dk, dv = A.ttt_backward_shared(s.cache.grads, q, k, v, att, datt, lse, s.mask, step_no, s.scaling)
-        dqkv = _rows(s.wqkv.dy_slot(slot_qkv, t), t, s.wqkv.w.shape[0], dev)
-        gemm._qkv_tokens(dqkv, (dq, dk, dv), s.positions, s.inv_freq, s.hq, s.hkv, s.d, s.offset,
-                         FO.table_scale_of(s.inv_freq))
-        dxin = gemm._project_back(dqkv, s.wqkv)
+        n, cache, mask = s.offset + 1, s.cache, s.mask
+        dk, dv = cache.grads.enter(n)
+        route, ws, right = gemm.backward_route(t, s.wqkv)
+        dqkv, dxin, dk, dv = _lib.native().ttt_backward(
+            q, cache.k, cache.v, att, datt, lse, mask.row_lo, dk, dv, s.wqkv.dy_slot(slot_qkv, t), s.positions, s.inv_freq,
+            s.offset, FO.table_scale_of(s.inv_freq), s.scaling, right, s.wqkv.w.shape[0], route, gemm.TAIL_PARTS,
+            gemm.workspace_for(q.device, ws), mask.ttt_step)
+        cache.grads.leave(n, dk, dv)
         tok_qkv = s.wqkv.defer(slot_qkv, dqkv, xin)
         d_gain_a = d_gain_b = None
         if s.first:
@@ -227,39 +225,11 @@ class NormedLayer:
                       self.wd.x_slot(t))
 
 
-def _head_norm_rope(tok, ld, out, passed, pos, s, gain, eps, t, heads, n_pass):
-    rstd = torch.empty(t, heads, device=out.device, dtype=torch.float32)
-    _lib.call("spx_head_norm_rope", tok, ld, out, t * s.d, passed, t * s.d, pos, s.inv_freq, gain, rstd, t, heads,
-              n_pass, s.d, 0, FO.table_scale_of(s.inv_freq), eps, _lib.stream_ptr(out.device))
-    return rstd
-
-
-def _head_norm_rope_backward(tok, ld, dout, dpass, pos, s, gain, rstd, grads, need_dw, dtok, ld_d, t, heads, n_pass):
-    """Writes ``dtok``; returns what autograd gets for the gain."""
-    dev = dout.device
-    st = _lib.stream_ptr(dev)
-    rows = t * heads
-    scratch, acc, shared = None, 0, None
-    if need_dw:
-        shared = grads.target(rows, s.d, dev) if grads is not None else None
-        scratch, acc = shared if shared is not None else (FO._dw_buffers(rows, s.d, dev)[0], 0)
-    _lib.call("spx_head_norm_rope_bwd", tok, ld, dout, t * s.d, dpass, t * s.d, pos, s.inv_freq, gain, rstd, dtok, ld_d,
-              scratch, acc, t, heads, n_pass, s.d, 0, FO.table_scale_of(s.inv_freq), st)
-    if not need_dw:
-        return None
-    if shared is not None:
-        return grads.mark(dev)
-    dw = torch.empty(s.d, device=dev, dtype=torch.bfloat16)
-    _lib.call("spx_rmsnorm_dweight", scratch, scratch.numel() // s.d, s.d, dw, st)
-    return dw
-
-
 def normed_forward(s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_post, gain_next):
     """``(y, normed, saved)`` as in ``step_forward``."""
     x2 = _flat(x)
     nq, h = x2.shape
     dev = x2.device
-    hq, hkv, d = s.hq, s.hkv, s.d
     slot_in, slot_o, slot_gu, slot_d = s.slots
     rstd_in = None
     if context is not None:
@@ -267,20 +237,15 @@ def normed_forward(s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_
         both = torch.cat((c2, _flat(n)))
         n2 = both[c2.shape[0]:]
         q_tok, kv_tok = gemm._project(n2, s.wq), gemm._project(both, s.wkv)
-        kv_at = kv_tok.data_ptr()
     else:
         rstd_in = torch.empty(nq, device=dev, dtype=torch.float32)
         both = n2 = _rows(slot_in, nq, h, dev)
         _lib.call("spx_rmsnorm_fwd", x2, x2.stride(0), gain_in, n2, h, rstd_in, nq, h, s.eps_in, _lib.stream_ptr(dev))
         q_tok = kv_tok = gemm._project(n2, s.wq)
-        kv_at = kv_tok.data_ptr() + 2 * hq * d
-    nk = both.shape[0]
-    q = torch.empty(1, hq, nq, d, device=dev, dtype=torch.bfloat16)
-    kv = torch.empty(2, 1, hkv, nk, d, device=dev, dtype=torch.bfloat16)
-    rq = _head_norm_rope(q_tok, q_tok.shape[1], q, None, s.q_pos, s, gain_q, s.eps_q, nq, hq, 0)
-    rk = _head_norm_rope(kv_at, kv_tok.shape[1], kv[0], kv[1], s.kv_pos, s, gain_k, s.eps_k, nk, hkv, hkv)
-    att = _rows(slot_o, nq, hq * d, dev)
-    lse = A.masked_forward_into(q, kv[0], kv[1], s.mask, s.scaling, att)
+    q, kv, rq, rk, att, lse = _lib.native().normed_forward(
+        q_tok, kv_tok, s.q_pos, s.kv_pos, s.inv_freq, gain_q, gain_k, slot_o, 0 if s.wkv is not None else s.hq * s.d, s.hq,
+        s.hkv, s.d, FO.table_scale_of(s.inv_freq), s.scaling, s.eps_q, s.eps_k,
+        *A.mask_arguments(s.mask, nq, both.shape[0]))
     y, normed, tail = _tail_forward(s, x2, att, gain_post, gain_next, slot_gu, slot_d, None)
     return y, normed, (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, *tail)
 
@@ -311,29 +276,24 @@ class _NormedLayer(torch.autograd.Function):
         (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, *tail, gain_in, gain_q, gain_k, gain_post,
          gain_next) = ctx.saved_tensors
         needs = ctx.needs_input_grad
-        hq, hkv, d = s.hq, s.hkv, s.d
         nq, h = n2.shape
         nk = both.shape[0]
         dev = n2.device
         grads_in, grads_q, grads_k, grads_post, grads_next = ctx.gain_grads
         da, datt, d_post, d_next, tok_o, tok_gu, tok_d = _tail_backward(
             s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads_next, needs[7:9], ctx.taken[2:])
-        dq, dk, dv = A.masked_backward(q, kv[0], kv[1], att, datt, lse, s.mask, s.scaling)
-        dq_tok = _rows(s.wq.dy_slot(ctx.taken[0], nq), nq, q_tok.shape[1], dev)
-        if s.wkv is not None:
-            dkv_tok = _rows(s.wkv.dy_slot(ctx.taken[1], nk), nk, kv_tok.shape[1], dev)
-            kv_at, dkv_at = kv_tok.data_ptr(), dkv_tok.data_ptr()
-        else:
-            dkv_tok = dq_tok
-            kv_at, dkv_at = kv_tok.data_ptr() + 2 * hq * d, dq_tok.data_ptr() + 2 * hq * d
-        d_gq = _head_norm_rope_backward(q_tok, q_tok.shape[1], dq, None, s.q_pos, s, gain_q, rq, grads_q, needs[5],
-                                        dq_tok, dq_tok.shape[1], nq, hq, 0)
-        d_gk = _head_norm_rope_backward(kv_at, kv_tok.shape[1], dk, dv, s.kv_pos, s, gain_k, rk, grads_k, needs[6],
-                                        dkv_at, dkv_tok.shape[1], nk, hkv, hkv)
+        sum_q, sum_k = _GainSum(grads_q, needs[5], nq * s.hq, s.d, dev), _GainSum(grads_k, needs[6], nk * s.hkv, s.d, dev)
+        two = s.wkv is not None
+        dq_tok, dkv_tok = _lib.native().normed_backward(
+            q_tok, kv_tok, q, kv, rq, rk, att, datt, lse, s.q_pos, s.kv_pos, s.inv_freq, gain_q, gain_k,
+            s.wq.dy_slot(ctx.taken[0], nq), s.wkv.dy_slot(ctx.taken[1], nk) if two else None, sum_q.scratch, sum_q.acc,
+            sum_k.scratch, sum_k.acc, 0 if two else s.hq * s.d, FO.table_scale_of(s.inv_freq), s.scaling,
+            *A.mask_arguments(s.mask, nq, nk))
+        d_gq, d_gk = sum_q.result(), sum_k.result()
         d_n = gemm._project_back(dq_tok, s.wq)
         tokens = [s.wq.defer(ctx.taken[0], dq_tok, n2)]
         d_context = d_in = None
-        if s.wkv is not None:
+        if two:
             d_both = gemm._project_back(dkv_tok, s.wkv)
             tokens.append(s.wkv.defer(ctx.taken[1], dkv_tok, both))
             d_n += d_both[nk - nq:]
