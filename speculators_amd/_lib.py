@@ -64,6 +64,7 @@ SIGNATURES["spx_rmsnorm_pair_bwd_partial"] = [_P, _I64, _P, _P, _I64, _P, _P, _I
                                               _I32, _P, _I32, _I64, _I64, _P]
 SIGNATURES["spx_rope_qkv"] = [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32,
                               _I64, _F, _P]
+SIGNATURES["spx_cat_bf16"] = [_P, _P, _P, _I32, _P, _P]
 SIGNATURES["spx_head_norm_rope"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I64, _F, _F, _P]
 SIGNATURES["spx_head_norm_rope_bwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I32, _I64, _I32, _I32,
                                         _I32, _I64, _F, _P]

@@ -134,6 +134,9 @@ PyMethodDef g_methods[] = {
     SPX_HOST("ttt_backward", spx_layer_ttt_backward)
     SPX_HOST("normed_forward", spx_layer_normed_forward)
     SPX_HOST("normed_backward", spx_layer_normed_backward)
+    SPX_HOST("product_tn", spx_layer_product_tn)
+    SPX_HOST("loss_step", spx_layer_loss_step)
+    SPX_HOST("cat_bf16", spx_layer_cat_bf16)
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},
     {nullptr, nullptr, 0, nullptr}};
 

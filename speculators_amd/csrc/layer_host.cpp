@@ -297,3 +297,95 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
   return tuple_of({dq_tok, dkv_tok});
   END_HANDLE_TH_ERRORS
 }
+
+// The weight gradient a^T b: (a [T, M], b [T, N], out or None, accumulate, fp32) -> [M, N]
+PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("product_tn", args, n, 5);
+  const Tensor &a = x.tensor(), &b = x.tensor();
+  Tensor out = x.maybe();
+  const int64_t accumulate = x.integer(), f32 = x.integer();
+  const int64_t t = a.size(0), m = a.size(1), cols = b.size(1);
+  if (!out.defined()) out = at::empty({m, cols}, a.options().dtype(f32 ? at::kFloat : at::kBFloat16));
+  check((f32 ? spx_gemm_bf16_tn_f32 : spx_gemm_bf16_tn)(in(a), a.stride(0), in(b), b.stride(0), out.mutable_data_ptr(),
+                                                        out.stride(0), m, cols, t, accumulate, stream_of(a)),
+        "spx_gemm_bf16_tn");
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// One TTT step's loss over bf16 logits in one read of the rows, with its masked mean: (op, logits, targets or None, known
+// lse_t, known argmax_t or None, mask, its kind, prev or None, its kind, acceptance counts or None (made and cleared here),
+// loss so far or None, step weight, term factor, scalars [8] or None: no mean) -> (total, row losses, argmax_draft,
+// argmax_target, lse_target, packed logits gradient, row map, live rows, row weights)
+PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("loss_step", args, n, 14);
+  const int64_t op = x.integer();
+  const Tensor &logits = x.tensor(), y = x.maybe(), known_lse = x.maybe(), known_arg = x.maybe(), &mask = x.tensor();
+  const int64_t mask_kind = x.integer();
+  const Tensor prev = x.maybe();
+  const int64_t prev_kind = x.integer();
+  const Tensor given = x.maybe(), total_in = x.maybe();
+  const double weight = x.number(), factor = x.number();
+  const Tensor out = x.maybe();
+  const int64_t rows = logits.size(0), vocab = logits.size(1);
+  const bool known = known_lse.defined();
+  void* const st = stream_of(logits);
+  const auto i32 = logits.options().dtype(at::kInt), f32 = logits.options().dtype(at::kFloat);
+  const Tensor map = at::empty({rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({5 * rows}, f32),
+               packed = at::empty({rows, vocab}, logits.options()), total = at::empty({}, f32);
+  int32_t* const row_map = map.mutable_data_ptr<int32_t>();
+  int32_t* const am = arg.mutable_data_ptr<int32_t>();
+  int32_t* const counts = given.defined() ? given.mutable_data_ptr<int32_t>() : am + 2 * rows;
+  float* const s = floats(stats);  // loss, lse_draft, lse_target, extra, row weights
+  float* const lse_t = known ? known_lse.mutable_data_ptr<float>() : s + 2 * rows;
+  int32_t* const am_t = known ? known_arg.mutable_data_ptr<int32_t>() : am + rows;
+  check(spx_mask_row_map(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows,
+                         given.defined() ? nullptr : counts, st),
+        "spx_mask_row_map");
+  check(spx_vocab_loss_step_fwd_grad(op, in(logits), logits.stride(0), y.defined() ? in(y) : nullptr,
+                                     y.defined() ? y.stride(0) : 0, rows, vocab, s, s + rows, lse_t, s + 3 * rows, am, am_t,
+                                     known, mask.const_data_ptr(), mask_kind,
+                                     prev.defined() ? prev.mutable_data_ptr() : nullptr, prev_kind, counts, row_map,
+                                     to(packed), vocab, st),
+        "spx_vocab_loss_step_fwd_grad");
+  if (out.defined())
+    check(spx_ttt_step_total(s, am, am_t, mask.const_data_ptr(), mask_kind, nullptr, 0, rows, weight, counts, factor,
+                             total_in.defined() ? total_in.const_data_ptr<float>() : nullptr, floats(total),
+                             floats(out), s + 4 * rows, st),
+          "spx_ttt_step_total");
+  return tuple_of({total, stats.narrow(0, 0, rows), arg.narrow(0, 0, rows), known ? known_arg : arg.narrow(0, rows, rows),
+                   known ? known_lse : stats.narrow(0, 2 * rows, rows), packed, map.narrow(0, 0, rows),
+                   map.narrow(0, rows, 1), stats.narrow(0, 4 * rows, rows)});
+  END_HANDLE_TH_ERRORS
+}
+
+// The row-wise concatenation of one to four matrices as one bf16 matrix
+PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n >= 1 && n <= 4, "cat_bf16 takes one to four tensors");
+  Args x("cat_bf16", args, n, n);
+  const void* src[4];
+  int64_t elements[4], rows = 0;
+  int32_t f32[4];
+  Tensor first;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const Tensor& t = x.tensor();
+    if (i == 0) first = t;
+    TORCH_CHECK_VALUE(t.is_contiguous() && t.dim() >= 1 && t.sizes().slice(1) == first.sizes().slice(1) &&
+                          t.device() == first.device() &&
+                          (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16),
+                      "contiguous bf16 or fp32 matrices of one width");
+    src[i] = t.const_data_ptr();
+    elements[i] = t.numel();
+    f32[i] = t.scalar_type() == at::kFloat;
+    rows += t.size(0);
+  }
+  auto shape = first.sizes().vec();
+  shape[0] = rows;
+  const Tensor out = at::empty(shape, first.options().dtype(at::kBFloat16).requires_grad(false));
+  check(spx_cat_bf16(src, elements, f32, n, out.mutable_data_ptr(), stream_of(first)), "spx_cat_bf16");
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}

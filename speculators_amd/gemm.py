@@ -43,7 +43,7 @@ def _split_workspace(device, numel: int) -> torch.Tensor:
     and grown on demand, so a TTT loop does not allocate hundreds of MB per step for a workspace the
     kernel leaves untouched whenever the device-side row count asks for one part.  Launches of one
     stream are ordered, so consecutive products may share it."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, _lib.stream_ptr(device))
     ws = _split_ws.get(key)
     if ws is None or ws.numel() < numel:
         ws = torch.empty(numel, device=device, dtype=torch.float32)
@@ -243,13 +243,13 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
             raise ValueError("accumulate needs the tensor to add to")
         if out_dtype not in (torch.bfloat16, torch.float32):
             raise ValueError("out_dtype must be bfloat16 or float32")
-        out = torch.empty(m, n, device=a.device, dtype=out_dtype)
     elif out.shape != (m, n) or out.dtype not in (torch.bfloat16, torch.float32) or out.stride(1) != 1:
         raise ValueError(f"out must be a bf16 or fp32 [{m}, {n}] tensor with unit column stride")
     # A small result with a long contraction leaves most of the chip idle (one workgroup per
     # 256 x 256 tile of the result): the contraction is then cut into row bands, every band's
     # product goes to an fp32 partial of its own (the grouped kernel with the bands as groups) and
     # the partials are summed in a fixed order
+    fp32 = (out_dtype if out is None else out.dtype) == torch.float32
     bands = _split_bands(t, m, n)
     if bands > 1 and max(a.stride(0), b.stride(0)) * 2 * (t + 256) < _MAX_SPAN:
         step = -(-t // bands)
@@ -258,19 +258,17 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
         _lib.call("spx_gemm_bf16_tn_grouped", a, a.stride(0), b, b.stride(0), part,
                   n, m * n, m, n, t, off, bands, 1, 0, _lib.stream_ptr(a.device))
         total = part.sum(0)
+        if out is None:
+            return total if fp32 else total.to(torch.bfloat16)
         if accumulate:
             total += out  # in fp32: what the result holds is added before the one rounding
         out.copy_(total)
         return out
-    entry = "spx_gemm_bf16_tn_f32" if out.dtype == torch.float32 else "spx_gemm_bf16_tn"
     # 32-bit byte offsets inside the kernel: a contraction that spans 2 GiB or more of an
     # operand is fed in bands of rows, every band after the first added to the result
     rows = max(_MAX_SPAN // (2 * max(a.stride(0), b.stride(0))) - 256, 1)
-    st = _lib.stream_ptr(a.device)
     for t0 in range(0, t, rows):
-        at, bt = a[t0:t0 + rows], b[t0:t0 + rows]
-        _lib.call(entry, at, at.stride(0), bt, bt.stride(0),
-                  out, out.stride(0), m, n, at.shape[0], int(accumulate or t0 > 0), st)
+        out = _lib.native().product_tn(a[t0:t0 + rows], b[t0:t0 + rows], out, accumulate or t0 > 0, fp32)
     return out
 
 

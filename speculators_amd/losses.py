@@ -44,9 +44,8 @@ class StepPass:
     ``d2t`` (int64 ``[Vd]``): the targets are FULL-vocabulary verifier rows and target element i
     is read at column ``i + d2t[i]`` while streaming; the draft-vocabulary rows come back in
     ``gathered`` (``[rows, Vd]``) for the later steps and the backward.
-    ``counts`` (int32 ``[3]``, zeroed -- or, with ``clear_counts``, cleared by the kernel that maps the rows in
-    front of the one-pass form, the only one that may then run): the acceptance chain is done row by row in the same pass
-    (``mask`` / ``prev`` are the step's 1-D views, ``prev`` is updated in place).
+    ``counts`` (int32 ``[3]``, zeroed; None in front of ``_loss_step``, which has its own): the acceptance chain is
+    done row by row in the same pass (``mask`` / ``prev`` are the step's 1-D views, ``prev`` is updated in place).
     ``grad_in_pass``: a promise of the caller that the reduction behind the row losses gives a row
     whose ``mask`` entry is zero the weight zero (the masked mean of ``compute_metrics`` does).  The
     head + loss node may then leave the gradient of the logits behind in the same row pass
@@ -59,7 +58,6 @@ class StepPass:
     prev: torch.Tensor | None = None
     counts: torch.Tensor | None = None
     grad_in_pass: bool = False
-    clear_counts: bool = False
 
 
 def fused_loss_forward(op: int, logits: torch.Tensor, targets: torch.Tensor, target_stats=None,
@@ -235,31 +233,25 @@ def _one_pass_ok(op, x, y, step) -> bool:
                          and y.data_ptr() % 16 == 0)
 
 
-def _loss_forward_with_grad(op, x, y, known, step):
-    """The row pass that also writes the unit-weight logits gradient of the unmasked rows, packed to
-    the front.  Returns ``(loss, lse_t, am_d, am_t, packed, row_map, count)``."""
-    rows, vocab = x.shape
-    dev = x.device
-    out = torch.empty(rows + 1, device=dev, dtype=torch.int32)
-    row_map, count = out[:rows], out[rows:]
-    _lib.call("spx_mask_row_map", step.mask, _lib.kind_code(step.mask), rows, row_map, count,
-              step.counts if step.clear_counts else None, _lib.stream_ptr(dev))
-    packed = torch.empty(rows, vocab, device=dev, dtype=torch.bfloat16)
-    stats = torch.empty(4, rows, device=dev, dtype=torch.float32)
-    arg = torch.empty(2, rows, device=dev, dtype=torch.int32)
-    lse_t, am_t = stats[2], arg[1]
+def _loss_step(op, x, y, known, step, mean=None, total_in=None):
+    """The row pass that also writes the unit-weight logits gradient of the unmasked rows, packed to the front, and
+    the masked mean behind it.  Returns ``(total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight)``."""
+    rows = x.shape[0]
+    lse_t = am_t = None
     if known is not None:
         lse_t, am_t = known[0].reshape(-1), known[1].reshape(-1)
         if lse_t.numel() != rows or am_t.numel() != rows or lse_t.stride(0) != 1 or am_t.stride(0) != 1:
             raise ValueError("target_stats must be contiguous [rows] tensors")
-    _lib.call(
-        "spx_vocab_loss_step_fwd_grad", op, x, x.stride(0), y,
-        y.stride(0) if y is not None else 0, rows, vocab, stats[0], stats[1],
-        lse_t, stats[3], arg[0], am_t, int(known is not None),
-        step.mask, _lib.kind_code(step.mask), step.prev,
-        _lib.kind_code(step.prev) if step.prev is not None else 0, step.counts,
-        row_map, packed, packed.stride(0), _lib.stream_ptr(dev))
-    return stats[0], lse_t, arg[0], am_t, packed, row_map, count
+    of_mean = (0.0, 0.0, None) if mean is None else (mean.weight, mean.factor, mean.out)
+    return _lib.native().loss_step(
+        op, x, y, lse_t, am_t, step.mask, _lib.kind_code(step.mask), step.prev,
+        _lib.kind_code(step.prev) if step.prev is not None else 0, step.counts, total_in, *of_mean)
+
+
+def _loss_forward_with_grad(op, x, y, known, step):
+    """``_loss_step`` without the mean: ``(loss, lse_t, am_d, am_t, packed, row_map, count)``."""
+    _, loss, am_d, am_t, lse_t, packed, row_map, count, _ = _loss_step(op, x, y, known, step)
+    return loss, lse_t, am_d, am_t, packed, row_map, count
 
 
 def _unpack_rows(packed: torch.Tensor, row_map: torch.Tensor, total_rows: int):
@@ -360,10 +352,8 @@ class _HeadStepLoss(torch.autograd.Function):
         xs = logits[:n_rows]
         ctx.one_pass = (known is not None or targets is not None) and _one_pass_ok(op, xs, targets, step)
         if ctx.one_pass:
-            step.counts = torch.empty(3, device=x2.device, dtype=torch.int32)
-            step.clear_counts = True
-            loss, lse_t, am_d, am_t, packed, row_map, count = _loss_forward_with_grad(op, xs, targets, known, step)
-            total, row_weight = mean.reduce(loss, am_d, am_t, step.counts, total_in)
+            total, _, am_d, am_t, lse_t, packed, row_map, count, row_weight = _loss_step(op, xs, targets, known, step, mean,
+                                                                                      total_in)
             ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
         else:
             step.counts = torch.zeros(3, device=x2.device, dtype=torch.int32)

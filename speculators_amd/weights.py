@@ -67,6 +67,10 @@ def _check_param_dtype(p: torch.Tensor):
 
 def _cat_bf16(params) -> torch.Tensor:
     """Row-wise concatenation of the parameters as one bf16 tensor (one pass: the copies cast)."""
+    if len(params) <= 4 and all(p.is_cuda and p.is_contiguous() and p.numel() % 8 == 0 and p.numel() > 0
+                                and p.data_ptr() % 16 == 0 and p.dtype in (torch.float32, torch.bfloat16)
+                                for p in params):
+        return _lib.native().cat_bf16(*params)
     if len(params) == 1:
         return params[0].detach().to(torch.bfloat16)
     rows = sum(p.shape[0] for p in params)

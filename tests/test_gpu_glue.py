@@ -486,3 +486,17 @@ def test_head_norm_rope_matches_the_separate_kernels(d, t, heads, n_pass):
     assert (dbuf[:, width:] == 5.0).all()
     _lib.call("spx_head_norm_rope_bwd", tok, tok.stride(0), dout, t * d, dpass if n_pass else None, t * d, pos, inv_freq,
               gain, rstd, dbuf, width + 8, None, 0, t, heads, n_pass, d, 3, 1.0, st)
+
+
+@pytest.mark.parametrize("rows,width,dtypes", [((1,), 8, "f"), ((3, 5), 40, "bf"), ((1024, 1, 2), 256, "ffb"),
+                                               ((513, 64, 64, 7), 1000, "bffb"), ((300,), 4096, "b"), ((8192, 8200), 4096, "bf")])
+def test_weights_are_concatenated_as_bf16(rows, width, dtypes):
+    """One launch for a merged weight of bf16 and fp32 parts: less than a workgroup, part boundaries inside one, four parts,
+    more than the last-level cache holds."""
+    from speculators_amd.weights import _cat_bf16
+
+    torch.manual_seed(width)
+    parts = [torch.randn(r, width, device="cuda").to(torch.float32 if k == "f" else torch.bfloat16)
+             for r, k in zip(rows, dtypes, strict=True)]
+    got = _cat_bf16(parts)
+    assert torch.equal(got, torch.cat([p.to(torch.bfloat16) for p in parts]))
