@@ -4,8 +4,12 @@ The layer (models/eagle3/model_definitions.py:14-110) is nine launches forward a
 eight nodes of their own they cost more host time (a node's forward and backward 20 us, and the views,
 slot look-ups and gradient checks between them) than the kernels take up to a thousand tokens: at 512
 tokens of the 1B shape a step of forward and backward was 0.61 ms of host time, 0.33 ms as one node.
-Nothing is computed differently: the same kernels in the same order, on the same buffers
-(``weights.Staged`` slots, the layer's K / V cache).
+The kernels, their order and their buffers (``weights.Staged`` slots, the layer's K / V cache) are those of the
+layer put together from its parts, with one difference: the anchored-block layer's k and v are one product.
+
+Whatever the backward reads beside the activations -- the compute weights, which for bf16 parameters are the
+parameters themselves, positions, rotary frequencies, mask bounds -- is saved with the node, so that autograd
+refuses a backward after one of them was changed in place.
 """
 
 from __future__ import annotations
@@ -38,6 +42,11 @@ class LayerStep:
         input buffers.  Asked for outside the node, where grad mode still says whether there is a graph."""
         self.slots = (self.wqkv.x_slot(t) if self.first else None, self.wo.x_slot(t), self.wgu.x_slot(t),
                       self.wd.x_slot(t), next_staged.x_slot(t) if next_staged is not None else None)
+
+
+    def constants(self):
+        """What the backward reads beside activations and gains, to be saved with the node."""
+        return (self.positions, self.inv_freq, self.mask.row_lo, self.wqkv.w, self.wo.w, self.wgu.w, self.wd.w)
 
 
 def _rows(t, rows, cols, device):
@@ -145,7 +154,7 @@ class _LayerStep(torch.autograd.Function):
         ctx.gain_grads = tuple(getattr(g, "spx_gain_grads", None) for g in (gain_a, gain_b, gain_post, gain_next))
         ctx.step = s
         ctx.shape = shape
-        ctx.save_for_backward(*saved, gain_a, gain_b, gain_post, gain_next)
+        ctx.save_for_backward(*saved, gain_a, gain_b, gain_post, gain_next, *s.constants())
         ctx.set_materialize_grads(False)
         return y.view(shape), normed.view(shape)
 
@@ -153,8 +162,9 @@ class _LayerStep(torch.autograd.Function):
     def backward(ctx, dy, dn):
         if dy is None and dn is None:
             return (None,) * 11
+        # (the weights come back for autograd's check alone: the products take them from the staged weights)
         (a2, b2, rstd_in, xin, q, att, lse, mid, stats, z, gu, act, y,
-         gain_a, gain_b, gain_post, gain_next) = ctx.saved_tensors
+         gain_a, gain_b, gain_post, gain_next, positions, inv_freq, row_lo, *_weights) = ctx.saved_tensors
         s = ctx.step
         needs = ctx.needs_input_grad
         t = y.shape[0]
@@ -167,7 +177,7 @@ class _LayerStep(torch.autograd.Function):
         dk, dv = cache.grads.enter(n)
         route, ws, right = gemm.backward_route(t, s.wqkv)
         dqkv, dxin, dk, dv = _lib.native().ttt_backward(
-            q, cache.k, cache.v, att, datt, lse, mask.row_lo, dk, dv, s.wqkv.dy_slot(slot_qkv, t), s.positions, s.inv_freq,
+            q, cache.k, cache.v, att, datt, lse, row_lo, dk, dv, s.wqkv.dy_slot(slot_qkv, t), positions, inv_freq,
             s.offset, FO.table_scale_of(s.inv_freq), s.scaling, right, s.wqkv.w.shape[0], route, gemm.TAIL_PARTS,
             gemm.workspace_for(q.device, ws), mask.ttt_step)
         cache.grads.leave(n, dk, dv)
@@ -208,6 +218,12 @@ class NormedLayer:
         self.hq, self.hkv, self.d = heads
         self.scaling, self.q_pos, self.kv_pos, self.inv_freq, self.mask = scaling, q_pos, kv_pos, inv_freq, mask
         self.slots, self.grad_slot = (None,) * 4, None
+
+    def constants(self, nq: int, nk: int):
+        """See ``LayerStep.constants``; the mask's bounds for ``nq`` query rows and ``nk`` keys come first."""
+        lo, hi, block_lo, block_hi, _, _ = A.mask_arguments(self.mask, nq, nk)
+        weights = (w.w for w in (self.wq, self.wkv, self.wo, self.wgu, self.wd) if w is not None)
+        return (lo, hi, block_lo, block_hi, self.q_pos, self.kv_pos, self.inv_freq, *weights)
 
     @staticmethod
     def takes(attention, inv_freq, kernel) -> bool:
@@ -264,7 +280,7 @@ class _NormedLayer(torch.autograd.Function):
         ctx.gain_grads = tuple(getattr(g, "spx_gain_grads", None) for g in gains)
         ctx.step, ctx.shape, ctx.n_inputs = s, x.shape, 9 + len(_tokens)
         ctx.context_shape = context.shape if context is not None else None
-        ctx.save_for_backward(*saved, *gains)
+        ctx.save_for_backward(*saved, *gains, *s.constants(n2.shape[0], both.shape[0]))
         ctx.set_materialize_grads(False)
         return y.view(x.shape), normed.view(x.shape)
 
@@ -273,8 +289,9 @@ class _NormedLayer(torch.autograd.Function):
         s = ctx.step
         if dy is None and dn is None:
             return (None,) * ctx.n_inputs
-        (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, *tail, gain_in, gain_q, gain_k, gain_post,
-         gain_next) = ctx.saved_tensors
+        (x2, rstd_in, both, n2, q_tok, kv_tok, rq, rk, q, kv, att, lse, mid, stats, z, gu, act, y, gain_in, gain_q, gain_k,
+         gain_post, gain_next, *bounds, q_pos, kv_pos, inv_freq) = ctx.saved_tensors[:30]
+        tail = (mid, stats, z, gu, act, y)
         needs = ctx.needs_input_grad
         nq, h = n2.shape
         nk = both.shape[0]
@@ -285,10 +302,10 @@ class _NormedLayer(torch.autograd.Function):
         sum_q, sum_k = _GainSum(grads_q, needs[5], nq * s.hq, s.d, dev), _GainSum(grads_k, needs[6], nk * s.hkv, s.d, dev)
         two = s.wkv is not None
         dq_tok, dkv_tok = _lib.native().normed_backward(
-            q_tok, kv_tok, q, kv, rq, rk, att, datt, lse, s.q_pos, s.kv_pos, s.inv_freq, gain_q, gain_k,
+            q_tok, kv_tok, q, kv, rq, rk, att, datt, lse, q_pos, kv_pos, inv_freq, gain_q, gain_k,
             s.wq.dy_slot(ctx.taken[0], nq), s.wkv.dy_slot(ctx.taken[1], nk) if two else None, sum_q.scratch, sum_q.acc,
-            sum_k.scratch, sum_k.acc, 0 if two else s.hq * s.d, FO.table_scale_of(s.inv_freq), s.scaling,
-            *A.mask_arguments(s.mask, nq, nk))
+            sum_k.scratch, sum_k.acc, 0 if two else s.hq * s.d, FO.table_scale_of(s.inv_freq), s.scaling, *bounds,
+            *A.mask_arguments(s.mask, nq, nk)[4:])
         d_gq, d_gk = sum_q.result(), sum_k.result()
         d_n = gemm._project_back(dq_tok, s.wq)
         tokens = [s.wq.defer(ctx.taken[0], dq_tok, n2)]

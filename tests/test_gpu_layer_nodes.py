@@ -1,0 +1,98 @@
+"""What the one-node decoder layers (``layer.py``) must keep of the layers put together from their parts: autograd's
+check of what a backward pass reads, the modules a program may hook or replace, parameters in any storage order."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FAMILIES = ("eagle3", "eagle3x2", "dflash", "mtp")
+LAYER = {"eagle3": "layers.0", "eagle3x2": "layers.1", "dflash": "layers.1", "mtp": "mtp_layers.0"}
+
+
+def _family(name):
+    """``(model, position_ids, forward)`` of a small bf16 model; ``forward()`` returns the loss."""
+    dev = "cuda"
+    g = torch.Generator().manual_seed(21)
+    torch.manual_seed(20)
+    kw = dict(hidden_size=256, num_attention_heads=4, num_key_value_heads=2, head_dim=64, intermediate_size=320)
+    t = 150
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=g).bfloat16().to(dev)
+
+    ids = torch.randint(0, 512, (1, t), generator=g).to(dev)
+    mask = (torch.rand(1, t, generator=g) < 0.7).to(dev)
+    doc = torch.arange(t).div(80, rounding_mode="floor").view(1, t).to(dev)
+    pos = (torch.arange(t) % 80).view(1, t).to(dev)
+    if name.startswith("eagle3"):
+        from speculators_amd.eagle3 import Eagle3Config, Eagle3DraftModel
+
+        model = Eagle3DraftModel(Eagle3Config(vocab_size=512, draft_vocab_size=512,
+                                              num_hidden_layers=2 if name.endswith("x2") else 1, **kw))
+        batch = dict(hidden_states=randn(1, t, 768), input_ids=ids, document_ids=doc, loss_mask=mask,
+                     position_ids=pos, verifier_last_hidden_states=randn(1, t, 256), ttt_steps=3)
+        at = 1
+    elif name == "dflash":
+        from speculators_amd.dflash import DFlashConfig, DFlashDraftModel
+
+        model = DFlashDraftModel(DFlashConfig(vocab_size=512, draft_vocab_size=512, num_aux=2, num_hidden_layers=2,
+                                              block_size=8, mask_token_id=7, **kw))
+        anchors = torch.tensor([3, 20, 41, 77, 90, 120], device=dev)
+        batch = dict(hidden_states=randn(1, t, 512), input_ids=ids, document_ids=doc, loss_mask=mask.float(),
+                     position_ids=pos, verifier_last_hidden_states=randn(1, t, 256),
+                     anchors=(anchors, torch.ones(6, dtype=torch.bool, device=dev)))
+        at = 1
+    else:
+        from speculators_amd.mtp import MTPConfig, MTPDraftModel
+
+        model = MTPDraftModel(MTPConfig(vocab_size=512, num_speculative_steps=2, **kw))
+        batch = dict(input_ids=ids, hidden_states=randn(1, t, 256), position_ids=pos, loss_mask=mask.float())
+        at = 1
+    model = model.to(dev).bfloat16()
+    return model, pos, lambda: model(**batch)[at]
+
+
+def _grads(model, forward):
+    model.zero_grad()
+    loss = forward()
+    loss.backward()
+    return loss.detach(), {n: p.grad for n, p in model.named_parameters() if p.grad is not None}
+
+
+def _same(got, want):
+    assert torch.equal(got[0], want[0])
+    assert got[1].keys() == want[1].keys() and len(want[1]) >= 8
+    for n, w in want[1].items():
+        assert torch.equal(got[1][n], w), n
+
+
+@pytest.mark.parametrize("family,what", [("eagle3", "self_attn.o_proj"), ("eagle3", "mlp.down_proj"),
+                                         ("eagle3", "positions"), ("eagle3x2", "mlp.down_proj"),
+                                         ("dflash", "self_attn.q_proj"), ("dflash", "self_attn.o_proj"),
+                                         ("dflash", "mlp.down_proj"), ("mtp", "self_attn.o_proj"),
+                                         ("mtp", "mlp.down_proj"), ("mtp", "positions")])
+def test_a_value_changed_in_place_before_the_backward_is_refused(family, what):
+    """bf16 parameters used as they lie and the caller's positions: changed between forward and backward they would give
+    the gradient of another function, and autograd says so -- also in the second pass over a retained graph."""
+    model, pos, forward = _family(family)
+    value = pos if what == "positions" else model.get_parameter(f"{LAYER[family]}.{what}.weight")
+    loss = forward()
+    loss.backward(retain_graph=True)  # unchanged: fine
+    with torch.no_grad():
+        value.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+
+
+def test_parameters_the_layer_reads_a_copy_of_may_change():
+    """The merged q/k/v and gate/up weights are copies: the gradient is that of the values the forward saw."""
+    model, _, forward = _family("eagle3")
+    want = _grads(model, forward)
+    model.zero_grad()
+    loss = forward()
+    with torch.no_grad():
+        model.layers[0].self_attn.k_proj.weight.mul_(2)
+        model.layers[0].mlp.up_proj.weight.zero_()
+    loss.backward()
+    _same((loss.detach(), {n: p.grad for n, p in model.named_parameters() if p.grad is not None}), want)
