@@ -82,6 +82,7 @@ def select_anchors(loss_mask: torch.Tensor, num_anchors: int, block_size: int):
     return anchors, ok
 
 
+@LY.passed_by
 class DFlashAttention(nn.Module):
     """q from the mask tokens; k/v from ``cat([context, mask tokens])``; per-head q/k
     RMSNorm; RoPE with the last q_len positions for q
@@ -127,10 +128,11 @@ class DFlashDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, stager)
 
     def _step(self, q_pos, kv_pos, inv_freq, mask, next_norm):
-        """The layer as one node (``layer.NormedLayer``), or None where it is put together from its parts: another
-        attention function or head size, or a graph in which some projection does not train."""
+        """The layer as one node (``layer.NormedLayer``), or None where it is put together from its parts: a hooked or
+        replaced module, another attention function or head size, or a graph in which some projection does not train."""
         att = self.self_attn
-        if next_norm is None or not LY.NormedLayer.takes(att, inv_freq, A.dflash_hip_attention_forward):
+        if (next_norm is None or not LY.untouched(att, self.mlp) or not LY.untouched(att.q_norm, att.k_norm)
+                or not LY.NormedLayer.takes(att, inv_freq, A.dflash_hip_attention_forward)):
             return None
         W = self._stager.get
         ws = (W(att.q_proj.weight), W(att.k_proj.weight, att.v_proj.weight), W(att.o_proj.weight),

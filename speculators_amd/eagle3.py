@@ -60,6 +60,7 @@ class Eagle3Config:
     embed_requires_grad: bool = False  # requires_grad of embed_tokens.weight (models/eagle3/core.py:68)
 
 
+@LY.passed_by
 class RMSNorm(nn.Module):
     """``stager``: the model's ``WeightStager`` (the gain is then read through it: bf16 compute copy
     of an fp32 master gain); None for a stand-alone norm on bf16 tensors."""
@@ -78,6 +79,7 @@ class RMSNorm(nn.Module):
         return FO.rms_norm(x, self.gain, self.eps)
 
 
+@LY.passed_by
 class Attention(nn.Module):
     def __init__(self, cfg: Eagle3Config, in_features: int, stager: WeightStager):
         super().__init__()
@@ -134,6 +136,7 @@ class Attention(nn.Module):
         return gemm.linear_staged(out.reshape(1, t, self.hq * self.d), W(self.o_proj.weight))
 
 
+@LY.passed_by
 class MLP(nn.Module):
     def __init__(self, cfg, stager: WeightStager):
         super().__init__()
@@ -178,12 +181,12 @@ class DecoderLayer(nn.Module):
 
     def _step(self, position_ids, pos_offset, inv_freq, cache, mask, next_norm, t, device):
         """The layer's next TTT step as one node (``layer.LayerStep``), or None where the layer is put
-        together from its parts: per-head norms, another attention function or head size, the normalised
-        hidden state as residual, or a graph in which some projection does not train."""
+        together from its parts: a hooked or replaced module, per-head norms, another attention function or
+        head size, the normalised hidden state as residual, or a graph in which some projection does not train."""
         att, cfg = self.self_attn, self.cfg
-        if (next_norm is None or att.qk_norm or att.attn_fn is not A.ttt_hip_attention_forward
-                or att.d not in A.KERNEL_HEAD_DIMS or not cache.get("steps")
-                or (self.first and cfg.norm_before_residual)):
+        if (next_norm is None or not LY.untouched(att, self.mlp) or att.qk_norm
+                or att.attn_fn is not A.ttt_hip_attention_forward or att.d not in A.KERNEL_HEAD_DIMS
+                or not cache.get("steps") or (self.first and cfg.norm_before_residual)):
             return None
         W = self._stager.get
         ws = (self._wqkv(), W(att.o_proj.weight), W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight),

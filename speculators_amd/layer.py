@@ -15,11 +15,27 @@ refuses a backward after one of them was changed in place.
 from __future__ import annotations
 
 import torch
+from torch.nn.modules import module as M
 
 from . import _lib
 from . import attention as A
 from . import fused_ops as FO
 from . import gemm
+
+
+def passed_by(cls):
+    """Class decorator: modules of ``cls`` are not called where their layer runs as one node."""
+    cls.forward_as_written = cls.forward
+    return cls
+
+
+def untouched(*modules) -> bool:
+    """Whether calling each of these modules would be its ``passed_by`` class's own ``forward`` and nothing else: no hook
+    on it or on every module, no other class, method or compiled call in its place."""
+    return not M._has_any_global_hook() and all(
+        type(m).forward is getattr(type(m), "forward_as_written", None) and "forward" not in m.__dict__
+        and m._compiled_call_impl is None and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                                                   or m._backward_pre_hooks) for m in modules)
 
 
 class LayerStep:

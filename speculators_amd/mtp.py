@@ -147,10 +147,12 @@ class MTPLayer(nn.Module):
 
     def _step(self, position_ids, inv_freq, mask):
         """What follows the input projection as one node (``layer.NormedLayer``), or None where it is put together
-        from its parts: no per-head norms, another attention function or head size, a rotary embedding over part
-        of the head, or a graph in which some projection does not train."""
+        from its parts: a hooked or replaced module, no per-head norms, another attention function or head size, a
+        rotary embedding over part of the head, or a graph in which some projection does not train."""
         att = self.self_attn
-        if not att.qk_norm or not LY.NormedLayer.takes(att, inv_freq, A.ttt_hip_attention_forward):
+        if (not LY.untouched(att, self.mlp, self.input_layernorm) or not att.qk_norm
+                or not LY.untouched(att.q_norm, att.k_norm)
+                or not LY.NormedLayer.takes(att, inv_freq, A.ttt_hip_attention_forward)):
             return None
         W = self._stager.get
         ws = (W(att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), None, W(att.o_proj.weight),

@@ -96,3 +96,72 @@ def test_parameters_the_layer_reads_a_copy_of_may_change():
         model.layers[0].mlp.up_proj.weight.zero_()
     loss.backward()
     _same((loss.detach(), {n: p.grad for n, p in model.named_parameters() if p.grad is not None}), want)
+
+
+CALLED = {"eagle3": ("self_attn", "mlp"), "eagle3x2": ("self_attn", "mlp"),
+          "dflash": ("self_attn", "mlp", "self_attn.q_norm", "self_attn.k_norm"),
+          "mtp": ("self_attn", "mlp", "input_layernorm", "self_attn.q_norm", "self_attn.k_norm")}
+
+
+@pytest.mark.parametrize("family,path", [(f, p) for f in FAMILIES for p in CALLED[f]])
+@pytest.mark.parametrize("way", ["hook", "pre_hook", "backward_hook", "instance", "replaced"])
+def test_modules_inside_a_layer_are_called_when_a_program_watches_them(family, path, way):
+    """Hooks on the modules inside a layer run, a replaced module or method is used, and what they change counts."""
+    model, _, forward = _family(family)
+    plain = forward().detach()
+    layer = model.get_submodule(LAYER[family])
+    module, calls = layer.get_submodule(path), []
+
+    def doubled(out):
+        calls.append(path)
+        return out * 2
+
+    if way == "hook":
+        module.register_forward_hook(lambda m, a, out: doubled(out))
+    elif way == "pre_hook":
+        module.register_forward_pre_hook(lambda m, a: (doubled(a[0]), *a[1:]))
+    elif way == "backward_hook":
+        module.register_full_backward_hook(lambda m, gi, go: calls.append(path))
+    elif way == "instance":
+        own = module.forward
+        module.forward = lambda *a: doubled(own(*a))
+    else:
+        class Wrapped(torch.nn.Module):
+            def __init__(self):
+                super().__init__()
+                self.inner = module
+
+            def __getattr__(self, name):
+                try:
+                    return super().__getattr__(name)
+                except AttributeError:
+                    return getattr(super().__getattr__("inner"), name)
+
+            def forward(self, *a):
+                return doubled(self.inner(*a))
+
+        parent, _, leaf = path.rpartition(".")
+        setattr(layer.get_submodule(parent) if parent else layer, leaf, Wrapped())
+    loss = forward()
+    loss.backward()
+    assert calls and torch.isfinite(loss)
+    # (an input norm of twice its input is the same norm)
+    norm_in = way == "pre_hook" and path.endswith("norm")
+    assert torch.equal(loss.detach(), plain) == (way == "backward_hook") or norm_in
+
+
+def test_global_hooks_and_a_class_method_replaced_see_the_inner_modules(monkeypatch):
+    from speculators_amd import eagle3 as E
+
+    model, _, forward = _family("eagle3")
+    plain = _grads(model, forward)
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, out: seen.append(type(m).__name__))
+    try:
+        _same(_grads(model, forward), plain)  # the layer put together from its parts is the same function
+    finally:
+        handle.remove()
+    assert seen.count("Attention") == seen.count("MLP") == 3
+    own = E.MLP.forward
+    monkeypatch.setattr(E.MLP, "forward", lambda self, x: own(self, x) * 2)
+    assert not torch.equal(forward().detach(), plain[0])
