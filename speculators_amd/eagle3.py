@@ -161,6 +161,7 @@ class _Prenormed(NamedTuple):
     normed: torch.Tensor
 
 
+@LY.passed_by
 class DecoderLayer(nn.Module):
     """Layer 0 carries the EAGLE3 first-layer changes
     (models/eagle3/model_definitions.py:14-110): q/k/v read ``cat([embeds, hidden])``
@@ -203,6 +204,13 @@ class DecoderLayer(nn.Module):
         att = self.self_attn
         return self._stager.get(att.q_proj.weight, att.k_proj.weight, att.v_proj.weight)
 
+    def _reader(self, next_layer):
+        """The staged weight that reads this layer's normed output as it is handed on, or None: into its input buffer
+        goes only what that weight's product will take (a place not taken is given to the next step)."""
+        if next_layer is None or not LY.untouched(self, next_layer, next_layer.self_attn) or next_layer.self_attn.qk_norm:
+            return None
+        return next_layer._wqkv()
+
     def forward(self, x, position_ids, pos_offset, inv_freq, cache, mask, next_norm=None, next_layer=None):
         """``x``: the hidden state, or for the first layer the pair ``(embeds, hidden)`` (their
         concatenation is what the reference passes).  With ``next_norm`` (the RMSNorm that
@@ -212,8 +220,7 @@ class DecoderLayer(nn.Module):
             one, two = x
             step = self._step(position_ids, pos_offset, inv_freq, cache, mask, next_norm, two.shape[1], two.device)
             if step is not None and one.dtype == two.dtype == torch.bfloat16:
-                step.take_slots(two.shape[1], None if next_layer is None or next_layer.self_attn.qk_norm
-                                else next_layer._wqkv())
+                step.take_slots(two.shape[1], self._reader(next_layer))
                 gains = (self.input_layernorm.gain, self.hidden_norm.gain) if self.first else (None, None)
                 return LY.run(step, one, two, *gains, self.post_attention_layernorm.gain, next_norm.gain)
         if self.first:

@@ -165,3 +165,27 @@ def test_global_hooks_and_a_class_method_replaced_see_the_inner_modules(monkeypa
     own = E.MLP.forward
     monkeypatch.setattr(E.MLP, "forward", lambda self, x: own(self, x) * 2)
     assert not torch.equal(forward().detach(), plain[0])
+
+
+def test_a_layer_output_replaced_by_a_hook_keeps_its_gradient():
+    """A forward hook on a layer that scales the normed state handed to the next layer: the scaling saves that state, which
+    later steps must not overwrite."""
+    from speculators_amd import eagle3 as E
+
+    losses, grads = [], []
+    for parts in (False, True):
+        model, _, forward = _family("eagle3x2")
+        scale = torch.nn.Parameter(torch.full((256,), 1.25, device="cuda", dtype=torch.bfloat16))
+        model.layers[0].register_forward_hook(lambda m, a, out: (out[0], out[1] * scale))
+        step = E.DecoderLayer._step
+        if parts:
+            E.DecoderLayer._step = lambda self, *a: None
+        try:
+            loss = forward()
+            loss.backward()
+        finally:
+            E.DecoderLayer._step = step
+        losses.append(loss.detach())
+        grads.append(scale.grad.float())
+    assert torch.equal(losses[0], losses[1])
+    assert (grads[0] - grads[1]).abs().max() <= 2e-2 * grads[1].abs().max()
