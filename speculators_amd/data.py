@@ -30,6 +30,7 @@ from __future__ import annotations
 
 import ctypes
 import json
+import math
 import os
 import queue
 import struct
@@ -95,8 +96,19 @@ class HiddenStatesFile:
         self.dtype = hs.dtype
 
     def data_offset(self, name: str) -> int:
-        """Where the bytes of a tensor start in the file."""
-        return self._data_offset + self.entries[name].begin
+        """Where the bytes of a tensor start in the file, once the header gives it as many as its shape needs."""
+        e = self.entries[name]
+        need = math.prod(e.shape) * torch.empty(0, dtype=e.dtype).element_size()
+        if e.end - e.begin != need:
+            raise ValueError(f"{self.path}: the header gives '{name}' {list(e.shape)} {e.end - e.begin} bytes, "
+                             f"its shape needs {need}")
+        return self._data_offset + e.begin
+
+    def check_size(self, nbytes: int) -> None:
+        """A file of ``nbytes`` bytes holds both tensors whole, whatever part of them is going to be read."""
+        for name in ("hidden_states", "token_ids"):
+            if self._data_offset + self.entries[name].end > nbytes:
+                raise OSError(f"{self.path}: the file ended before its tensor '{name}' did")
 
     def read_into(self, name: str, dst: torch.Tensor) -> None:
         """Fill ``dst`` (contiguous CPU tensor of the entry's dtype and element count)."""
@@ -300,6 +312,7 @@ class BatchPacker:
                 if isinstance(hs, HiddenStatesFile):
                     fd = os.open(hs.path, os.O_RDONLY)
                     fds.append(fd)
+                    hs.check_size(os.fstat(fd).st_size)
                     hs_seg.append((None, dst, hs.data_offset("hidden_states"), n, fd))
                     if hs.entries["token_ids"].dtype == torch.int64:
                         ids_seg.append((None, ids0 + 8 * at, hs.data_offset("token_ids"), 8 * keep, fd))

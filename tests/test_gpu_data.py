@@ -170,6 +170,31 @@ def test_pack_large_batch_from_files_and_memory(tmp_path):
     _check(packer([raws[1]]), _want([raws[1]], max_len, hidden, layers, "eagle3"))
 
 
+@pytest.mark.parametrize("case", ["states short", "states long", "ids short", "ids long", "ends early", "ends early, cut"])
+def test_files_whose_header_or_length_is_wrong_are_refused(tmp_path, case):
+    """Byte ranges in the header that disagree with a tensor's shape, and a file that ends inside a tensor -- behind the
+    rows that fit the batch, too: an error, nothing of a neighbouring tensor in the batch, and a packer that goes on."""
+    import json
+
+    from speculators_amd.data import BatchPacker, HiddenStatesFile
+
+    g = torch.Generator().manual_seed(8)
+    raw = _raw(12, 3, 64, g, torch.bfloat16)
+    hs, ids = raw["hidden_states"].view(torch.int16).numpy().tobytes(), raw["token_ids"].numpy().tobytes()
+    n_hs = len(hs) + {"states short": -128, "states long": 128}.get(case, 0)
+    n_ids = len(ids) + {"ids short": -8, "ids long": 8}.get(case, 0)
+    header = json.dumps({"hidden_states": {"dtype": "BF16", "shape": [12, 4, 64], "data_offsets": [0, n_hs]},
+                         "token_ids": {"dtype": "I64", "shape": [12], "data_offsets": [n_hs, n_hs + n_ids]}}).encode()
+    blob = len(header).to_bytes(8, "little") + header + hs + ids + bytes(256)
+    early = case.startswith("ends early")
+    (tmp_path / "a.safetensors").write_bytes(blob[:-256 - 40] if early else blob)
+    # (the last case: only the first rows of the document are staged, and those are in the file)
+    packer = BatchPacker(6 if case.endswith("cut") else 32, 64, 3)
+    with pytest.raises(OSError if early else ValueError):
+        packer([{"hidden_states": HiddenStatesFile(tmp_path / "a.safetensors"), "loss_mask": raw["loss_mask"]}])
+    _check(packer([raw]), _want([raw], packer.max_len, 64, 3, "eagle3"))
+
+
 def test_loader_hands_worker_errors_to_the_caller(tmp_path):
     from speculators_amd.data import BatchPacker, PackedBatchLoader
 
