@@ -82,6 +82,16 @@ def _cat_bf16(params) -> torch.Tensor:
     return out
 
 
+def _as_it_lies(p: torch.Tensor) -> torch.Tensor:
+    """A bf16 parameter used alone: itself -- or a copy in rows of aligned chunks where it is a matrix stored otherwise
+    (column by column, at an odd address, with an odd or overlapping row stride): the GEMM kernels take none of these."""
+    w = p.detach()
+    if w.dim() == 2 and w.shape[1] % 8 == 0 and (w.stride(1) != 1 or w.stride(0) % 8 or w.stride(0) < w.shape[1]
+                                                 or w.data_ptr() % 16):
+        return w.clone(memory_format=torch.contiguous_format)
+    return w
+
+
 def transposed_copy(w: torch.Tensor) -> torch.Tensor:
     """``w.transpose(-1, -2)`` as a new contiguous tensor; a stack ``[E, N, K]`` is transposed
     matrix by matrix.  On the library's kernel where its alignment rules hold."""
@@ -291,7 +301,7 @@ class _Stage(torch.autograd.Function):
         ctx.rows = [p.shape[0] for p in params]
         ctx.dtypes = [p.dtype for p in params]
         if len(params) == 1 and params[0].dtype == torch.bfloat16:
-            w = params[0].detach()
+            w = _as_it_lies(params[0])
         else:
             w = _cat_bf16(params)
         token = _lib.zero(w.device).expand(w.shape)
@@ -381,7 +391,7 @@ class WeightStager:
             fkey = tuple((p.data_ptr(), p._version, p.dtype) for p in params)
             kept = self._frozen.get(key)
             if kept is None or kept[0] != fkey:
-                w = params[0].detach() if len(params) == 1 and params[0].dtype == torch.bfloat16 \
+                w = _as_it_lies(params[0]) if len(params) == 1 and params[0].dtype == torch.bfloat16 \
                     else _cat_bf16(params)
                 kept = (fkey, Staged(w, rows_of))
                 if not any(p.requires_grad for p in params):

@@ -189,3 +189,33 @@ def test_a_layer_output_replaced_by_a_hook_keeps_its_gradient():
         grads.append(scale.grad.float())
     assert torch.equal(losses[0], losses[1])
     assert (grads[0] - grads[1]).abs().max() <= 2e-2 * grads[1].abs().max()
+
+
+LONE = {"eagle3": ("self_attn.o_proj", "mlp.down_proj"),
+        "dflash": ("self_attn.q_proj", "self_attn.o_proj", "mlp.down_proj"),
+        "mtp": ("input_proj", "self_attn.o_proj", "mlp.down_proj")}
+
+
+@pytest.mark.parametrize("family", sorted(LONE))
+@pytest.mark.parametrize("order", ["columns", "odd_address", "odd_rows", "wide_rows"])
+def test_bf16_weights_in_any_storage_order(family, order):
+    """Weights that lie column by column, at an address or with a row stride the kernels do not take, or with a gap between
+    the rows: the same results, bit for bit."""
+    model, _, forward = _family(family)
+    want = _grads(model, forward)
+    layer = model.get_submodule(LAYER[family])
+    for path in LONE[family]:
+        lin = layer.get_submodule(path)
+        w = lin.weight.detach()
+        n, k = w.shape
+        if order == "columns":
+            new = w.t().contiguous().t()
+        elif order == "odd_address":
+            new = torch.empty(n * k + 1, device=w.device, dtype=w.dtype)[1:].view(n, k).copy_(w)
+        else:
+            new = torch.empty(n, k + (3 if order == "odd_rows" else 64), device=w.device, dtype=w.dtype)[:, :k].copy_(w)
+        assert torch.equal(new, w) and new.stride() + (new.data_ptr() % 16,) != w.stride() + (0,)
+        lin.weight = torch.nn.Parameter(new)
+    _same(_grads(model, forward), want)
+    with torch.no_grad():
+        assert torch.isfinite(forward())
