@@ -265,8 +265,12 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
         out.copy_(total)
         return out
     # 32-bit byte offsets inside the kernel: a contraction that spans 2 GiB or more of an
-    # operand is fed in bands of rows, every band after the first added to the result
+    # operand is fed in bands of rows, every band after the first added to the result.  A bf16 result of several
+    # bands is formed in fp32 and rounded once, like that of one
     rows = max(_MAX_SPAN // (2 * max(a.stride(0), b.stride(0))) - 256, 1)
+    if t > rows and not fp32:
+        total = gemm_tn(a, b, out.float() if accumulate else None, accumulate, torch.float32)
+        return total.to(torch.bfloat16) if out is None else out.copy_(total)
     for t0 in range(0, t, rows):
         out = _lib.native().product_tn(a[t0:t0 + rows], b[t0:t0 + rows], out, accumulate or t0 > 0, fp32)
     return out

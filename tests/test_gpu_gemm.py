@@ -518,3 +518,24 @@ def test_product_on_the_tile_its_size_asks_for(form, m, n, k):
     if not big:
         some = run(torch.tensor([live], dtype=torch.int32, device="cuda"), live)
         assert torch.equal(some.view(torch.int16), full[:live].view(torch.int16))
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_tn_in_row_bands_rounds_a_bf16_result_once(accumulate, monkeypatch):
+    """Operands too large for one launch are fed in bands of rows (forced here by a small limit: 20 bands).  The bands are
+    added in fp32: a bf16 result is the exact one to half a unit in its last place (2^-8 relative at a mantissa of one) and
+    what 1200 fp32 additions may lose."""
+    from speculators_amd import gemm
+
+    t, m, n = 1200, 264, 136
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = (1 + torch.rand(t, m, device="cuda", generator=g)).bfloat16()  # (one sign: no cancellation)
+    b = (1 + torch.rand(t, n, device="cuda", generator=g)).bfloat16()
+    base = (100 * torch.rand(m, n, device="cuda", generator=g)).bfloat16()
+    monkeypatch.setattr(gemm, "_MAX_SPAN", 2 * m * (256 + 60))
+    out = gemm.gemm_tn(a, b, base.clone(), accumulate=True) if accumulate else gemm.gemm_tn(a, b)
+    assert out.dtype == torch.bfloat16
+    want = a.double().t() @ b.double() + (base.double() if accumulate else 0)
+    assert ((out.double() - want).abs() / want).max().item() <= 2 ** -8 + 1200 * 2 ** -24
+    f32 = gemm.gemm_tn(a, b, out_dtype=torch.float32)
+    assert ((f32.double() - a.double().t() @ b.double()).abs() / want).max().item() <= 1200 * 2 ** -24
