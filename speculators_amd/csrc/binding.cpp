@@ -4,7 +4,8 @@
 // pointer), or a HIP tensor where the C function takes a pointer -- converts them without an intermediate object, calls
 // the function and raises SpxError when its status is not zero.  A call costs what the launch costs: 6.9 us through
 // ctypes (argument objects, the foreign call, the status check in Python), 3 us here; a training step of a small draft
-// makes a hundred of them.
+// makes a hundred of them.  Entry points that launch are called without the interpreter's lock: a launch that waits for
+// room in the queue, or a file that is read, does not hold up the program's other threads (the batch producer's).
 
 #include <Python.h>
 
@@ -51,7 +52,7 @@ bool convert(PyObject* o, T& out) {
   }
 }
 
-template <bool kUnlock, auto kFn, typename R, typename... A>
+template <bool kStatus, auto kFn, typename R, typename... A>
 PyObject* call_with(const char* name, PyObject* const* args, Py_ssize_t n, R (*)(A...)) {
   constexpr Py_ssize_t kArgs = sizeof...(A);
   if (n != kArgs) {
@@ -64,7 +65,7 @@ PyObject* call_with(const char* name, PyObject* const* args, Py_ssize_t n, R (*)
   }(std::make_index_sequence<sizeof...(A)>{});
   if (!ok) return nullptr;
   R r;
-  if constexpr (kUnlock) {
+  if constexpr (kStatus) {
     Py_BEGIN_ALLOW_THREADS
     r = std::apply(kFn, v);
     Py_END_ALLOW_THREADS
@@ -77,9 +78,9 @@ PyObject* call_with(const char* name, PyObject* const* args, Py_ssize_t n, R (*)
 }
 
 // kStatus: the result is a status, not a value
-template <bool kStatus, bool kUnlock, auto kFn>
+template <bool kStatus, auto kFn>
 PyObject* entry(const char* name, PyObject* const* args, Py_ssize_t n) {
-  PyObject* r = call_with<kUnlock, kFn>(name, args, n, kFn);
+  PyObject* r = call_with<kStatus, kFn>(name, args, n, kFn);
   if constexpr (kStatus) {
     if (!r) return nullptr;
     const long rc = PyLong_AsLong(r);
@@ -95,19 +96,14 @@ PyObject* entry(const char* name, PyObject* const* args, Py_ssize_t n) {
 
 #define SPX_STATUS(fn)                                                                       \
   static PyObject* py_##fn(PyObject*, PyObject* const* args, Py_ssize_t n) {                \
-    return entry<true, false, &fn>(#fn, args, n);                                           \
-  }
-#define SPX_UNLOCKED(fn)                                                                     \
-  static PyObject* py_##fn(PyObject*, PyObject* const* args, Py_ssize_t n) {                \
-    return entry<true, true, &fn>(#fn, args, n);                                            \
+    return entry<true, &fn>(#fn, args, n);                                                  \
   }
 #define SPX_VALUE(fn)                                                                        \
   static PyObject* py_##fn(PyObject*, PyObject* const* args, Py_ssize_t n) {                \
-    return entry<false, false, &fn>(#fn, args, n);                                          \
+    return entry<false, &fn>(#fn, args, n);                                                 \
   }
 #include "binding_list.h"
 #undef SPX_STATUS
-#undef SPX_UNLOCKED
 #undef SPX_VALUE
 
 PyObject* set_error(PyObject*, PyObject* cls) {
@@ -121,7 +117,6 @@ PyObject* set_error(PyObject*, PyObject* cls) {
 #define SPX_HOST(name, fn) \
   {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&fn)), METH_FASTCALL, nullptr},
 #define SPX_STATUS(fn) SPX_ROW(fn)
-#define SPX_UNLOCKED(fn) SPX_ROW(fn)
 #define SPX_VALUE(fn) SPX_ROW(fn)
 PyMethodDef g_methods[] = {
 #include "binding_list.h"

@@ -2,6 +2,8 @@
 #pragma once
 #include <Python.h>
 
+#include <utility>
+
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -28,6 +30,20 @@ inline void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t
 inline void check(int rc, const char* name) {
   if (rc != 0) fail("%s failed (%ld): %s", name, rc, spx_last_error());
 }
+// The interpreter's lock given up, from the construction on until lock() or the end of the scope (by an exception, too).
+// No Python object is touched in between; the tensors of the call's arguments stay, its caller holds them.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { lock(); }
+  void lock() {
+    if (state_) PyEval_RestoreThread(std::exchange(state_, nullptr));
+  }
+
+ private:
+  PyThreadState* state_;
+};
 inline void need_hip(const Tensor& t) {
   if (!t.is_cuda()) fail("%s", "libspx_hip works on HIP device tensors only (got a CPU tensor)");
 }

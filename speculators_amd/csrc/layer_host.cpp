@@ -39,7 +39,12 @@ struct Args {
   }
 };
 
-PyObject* tuple_of(std::initializer_list<Tensor> ts) {
+PyObject* wrapped(Unlocked& released, const Tensor& t) {
+  released.lock();
+  return THPVariable_Wrap(t);
+}
+PyObject* tuple_of(Unlocked& released, std::initializer_list<Tensor> ts) {
+  released.lock();
   PyObject* const out = PyTuple_New(ts.size());
   Py_ssize_t i = 0;
   for (const Tensor& t : ts) PyTuple_SET_ITEM(out, i++, THPVariable_Wrap(t));
@@ -94,7 +99,9 @@ PyObject* spx_layer_product(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t route = x.integer();
   const Tensor &a = x.tensor(), &b = x.tensor(), live = x.maybe();
   const int64_t parts = x.integer();
-  return THPVariable_Wrap(Products{parts, x.maybe()}(route, a, b, live));
+  const Products product{parts, x.maybe()};
+  Unlocked released;
+  return wrapped(released, product(route, a, b, live));
   END_HANDLE_TH_ERRORS
 }
 
@@ -108,6 +115,7 @@ PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n)
   const double eps_post = x.number(), eps_next = x.number();
   const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
+  Unlocked released;
   const int64_t t = residual.size(0), h = residual.size(1), f = wgu.size(0) / 2;
   void* const st = stream_of(residual);
   const Tensor stats = at::empty({2, t}, residual.options().dtype(at::kFloat));
@@ -123,7 +131,7 @@ PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n)
   const Tensor y = at::empty({t, h}, residual.options()), normed = rows_or_new(slot_next, t, h, residual);
   check(spx_add_rmsnorm_fwd(in(mid), h, in(m), h, to(y), h, in(gain_next), to(normed), h, rstd + t, t, h, eps_next, st),
         "spx_add_rmsnorm_fwd");
-  return tuple_of({mid, stats, z, gu, act, y, normed});
+  return tuple_of(released, {mid, stats, z, gu, act, y, normed});
   END_HANDLE_TH_ERRORS
 }
 
@@ -141,6 +149,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   const int64_t acc_next = x.integer();
   const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
+  Unlocked released;
   const int64_t t = y.size(0), h = y.size(1), f = gu.size(1) / 2;
   void* const st = stream_of(y);
   const float* const rstd = floats(stats);
@@ -162,7 +171,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   check(spx_rmsnorm_bwd_partial(in(mid), h, in(gain_post), in(dz), h, in(dm), h, rstd, to(da), h, floats(scratch_post),
                                 acc_post, t, h, st),
         "spx_rmsnorm_bwd_partial");
-  return tuple_of({dm, dgu, da, product(r_o, da, bo)});
+  return tuple_of(released, {dm, dgu, da, product(r_o, da, bo)});
   END_HANDLE_TH_ERRORS
 }
 
@@ -176,6 +185,7 @@ PyObject* spx_layer_ttt_forward(PyObject*, PyObject* const* args, Py_ssize_t n) 
   const double table_scale = x.number(), scaling = x.number();
   const int64_t route = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
+  Unlocked released;
   const int64_t t = xin.size(0), at = offset * t * d;
   TORCH_CHECK_VALUE(k.size(2) >= (offset + 1) * t && row_lo.numel() == t && pos.numel() == t && step == offset,
                     "the layer's cache, mask and positions do not fit step ", offset, " of ", t, " tokens");
@@ -188,7 +198,7 @@ PyObject* spx_layer_ttt_forward(PyObject*, PyObject* const* args, Py_ssize_t n) 
         "spx_rope_qkv");
   const Tensor att = rows_or_new(slot, t, hq * d, xin);
   const Tensor lse = attention_forward(q, k, v, Mask{row_lo, {}, {}, {}, t, step}, scaling, att);
-  return tuple_of({q, att, lse});
+  return tuple_of(released, {q, att, lse});
   END_HANDLE_TH_ERRORS
 }
 
@@ -208,6 +218,7 @@ PyObject* spx_layer_ttt_backward(PyObject*, PyObject* const* args, Py_ssize_t n)
   const int64_t n_qkv = x.integer(), route = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
   const int64_t step = x.integer();
+  Unlocked released;
   const int64_t hq = q.size(1), t = q.size(2), d = q.size(3), hkv = k.size(1), keys = (offset + 1) * t, at = offset * t * d;
   void* const st = stream_of(q);
   const bool add = dk.defined();
@@ -229,7 +240,7 @@ PyObject* spx_layer_ttt_backward(PyObject*, PyObject* const* args, Py_ssize_t n)
                      pos.const_data_ptr<int64_t>(), inv_freq.const_data_ptr<float>(), t, hq, hkv, d,
                      2 * inv_freq.numel(), 1, offset, table_scale, st),
         "spx_rope_qkv");
-  return tuple_of({dqkv, product(route, dqkv, w), dk, dv});
+  return tuple_of(released, {dqkv, product(route, dqkv, w), dk, dv});
   END_HANDLE_TH_ERRORS
 }
 
@@ -244,6 +255,7 @@ PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t 
   const double table_scale = x.number(), scaling = x.number(), eps_q = x.number(), eps_k = x.number();
   const Tensor &lo = x.tensor(), hi = x.maybe(), blo = x.maybe(), bhi = x.maybe();
   const int64_t T = x.integer(), step = x.integer();
+  Unlocked released;
   const int64_t nq = q_tok.size(0), nk = kv_tok.size(0);
   TORCH_CHECK_VALUE(q_pos.numel() == nq && kv_pos.numel() == nk, "positions of ", nq, " and ", nk, " rows");
   void* const st = stream_of(q_tok);
@@ -261,7 +273,7 @@ PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t 
         "spx_head_norm_rope");
   const Tensor att = rows_or_new(slot, nq, hq * d, q_tok);
   const Tensor lse = attention_forward(q, k, v, Mask{lo, hi, blo, bhi, T, step}, scaling, att);
-  return tuple_of({q, kv, rq, rk, att, lse});
+  return tuple_of(released, {q, kv, rq, rk, att, lse});
   END_HANDLE_TH_ERRORS
 }
 
@@ -279,6 +291,7 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
   const double table_scale = x.number(), scaling = x.number();
   const Tensor &lo = x.tensor(), hi = x.maybe(), blo = x.maybe(), bhi = x.maybe();
   const int64_t T = x.integer(), step = x.integer();
+  Unlocked released;
   const int64_t hq = q.size(1), nq = q.size(2), d = q.size(3), hkv = kv.size(2), nk = kv.size(3);
   void* const st = stream_of(q);
   const auto [dq, dk, dv] = attention_backward(q, kv.select(0, 0), kv.select(0, 1), att, datt, lse,
@@ -294,7 +307,7 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
                                kv_pos.const_data_ptr<int64_t>(), f, in(gain_k), floats(rk), to(dkv_tok) + kv_column,
                                dkv_tok.stride(0), floats(scratch_k), acc_k, nk, hkv, hkv, d, 0, table_scale, st),
         "spx_head_norm_rope_bwd");
-  return tuple_of({dq_tok, dkv_tok});
+  return tuple_of(released, {dq_tok, dkv_tok});
   END_HANDLE_TH_ERRORS
 }
 
@@ -305,12 +318,13 @@ PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor &a = x.tensor(), &b = x.tensor();
   Tensor out = x.maybe();
   const int64_t accumulate = x.integer(), f32 = x.integer();
+  Unlocked released;
   const int64_t t = a.size(0), m = a.size(1), cols = b.size(1);
   if (!out.defined()) out = at::empty({m, cols}, a.options().dtype(f32 ? at::kFloat : at::kBFloat16));
   check((f32 ? spx_gemm_bf16_tn_f32 : spx_gemm_bf16_tn)(in(a), a.stride(0), in(b), b.stride(0), out.mutable_data_ptr(),
                                                         out.stride(0), m, cols, t, accumulate, stream_of(a)),
         "spx_gemm_bf16_tn");
-  return THPVariable_Wrap(out);
+  return wrapped(released, out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -329,6 +343,7 @@ PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor given = x.maybe(), total_in = x.maybe();
   const double weight = x.number(), factor = x.number();
   const Tensor out = x.maybe();
+  Unlocked released;
   const int64_t rows = logits.size(0), vocab = logits.size(1);
   const bool known = known_lse.defined();
   void* const st = stream_of(logits);
@@ -355,9 +370,10 @@ PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
                              total_in.defined() ? total_in.const_data_ptr<float>() : nullptr, floats(total),
                              floats(out), s + 4 * rows, st),
           "spx_ttt_step_total");
-  return tuple_of({total, stats.narrow(0, 0, rows), arg.narrow(0, 0, rows), known ? known_arg : arg.narrow(0, rows, rows),
-                   known ? known_lse : stats.narrow(0, 2 * rows, rows), packed, map.narrow(0, 0, rows),
-                   map.narrow(0, rows, 1), stats.narrow(0, 4 * rows, rows)});
+  return tuple_of(released, {total, stats.narrow(0, 0, rows), arg.narrow(0, 0, rows),
+                             known ? known_arg : arg.narrow(0, rows, rows),
+                             known ? known_lse : stats.narrow(0, 2 * rows, rows), packed, map.narrow(0, 0, rows),
+                             map.narrow(0, rows, 1), stats.narrow(0, 4 * rows, rows)});
   END_HANDLE_TH_ERRORS
 }
 
@@ -382,10 +398,11 @@ PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
     f32[i] = t.scalar_type() == at::kFloat;
     rows += t.size(0);
   }
+  Unlocked released;
   auto shape = first.sizes().vec();
   shape[0] = rows;
   const Tensor out = at::empty(shape, first.options().dtype(at::kBFloat16).requires_grad(false));
   check(spx_cat_bf16(src, elements, f32, n, out.mutable_data_ptr(), stream_of(first)), "spx_cat_bf16");
-  return THPVariable_Wrap(out);
+  return wrapped(released, out);
   END_HANDLE_TH_ERRORS
 }

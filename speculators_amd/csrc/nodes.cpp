@@ -161,8 +161,12 @@ PyObject* spx_node_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t T = PyLong_AsLongLong(args[7]), step = PyLong_AsLongLong(args[8]);
   const double scaling = PyFloat_AsDouble(args[9]);
   if (PyErr_Occurred()) return nullptr;
-  return THPVariable_Wrap(Attention::apply(q, k, v, tensor(args[3]), tensor_or_none(args[4]),
-                                           tensor_or_none(args[5]), tensor_or_none(args[6]), T, step, scaling));
+  const Tensor& lo = tensor(args[3]);
+  const auto hi = tensor_or_none(args[4]), block_lo = tensor_or_none(args[5]), block_hi = tensor_or_none(args[6]);
+  Unlocked released;
+  const Tensor out = Attention::apply(q, k, v, lo, hi, block_lo, block_hi, T, step, scaling);
+  released.lock();
+  return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -174,6 +178,9 @@ PyObject* spx_node_row_loss(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor &x = tensor(args[1]), &y = tensor(args[2]);
   TORCH_CHECK_VALUE(x.sizes() == y.sizes(), "logits ", x.sizes(), " and targets ", y.sizes(), " differ");
   need_hip(x); need_hip(y);
-  return THPVariable_Wrap(RowLoss::apply(x, y, op));
+  Unlocked released;
+  const Tensor out = RowLoss::apply(x, y, op);
+  released.lock();
+  return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import functools
 import os
+import threading
 
 import torch
 
@@ -35,19 +36,27 @@ TAIL_PARTS = int(os.environ.get("SPX_GEMM_TAIL_PARTS", "4"))
 if not 1 <= TAIL_PARTS <= 8:
     raise ValueError(f"SPX_GEMM_TAIL_PARTS must be 1 .. 8, got {TAIL_PARTS}")
 
-_split_ws: dict = {}
+class _Workspaces(threading.local):
+    """One thread's buffers, by (device, stream); they go with the thread."""
+
+    def __init__(self):
+        self.held: dict = {}
+
+
+_workspaces = _Workspaces()
 
 
 def _split_workspace(device, numel: int) -> torch.Tensor:
-    """The fp32 partials of a product cut along its contraction: one buffer per (device, stream), kept
+    """The fp32 partials of a product cut along its contraction: one buffer per (thread, device, stream), kept
     and grown on demand, so a TTT loop does not allocate hundreds of MB per step for a workspace the
-    kernel leaves untouched whenever the device-side row count asks for one part.  Launches of one
-    stream are ordered, so consecutive products may share it."""
+    kernel leaves untouched whenever the device-side row count asks for one part.  The launches of one thread
+    on one stream are ordered, so consecutive products may share it; another thread's may come between the launches of a
+    product."""
+    held = _workspaces.held
     key = (device.index, _lib.stream_ptr(device))
-    ws = _split_ws.get(key)
+    ws = held.get(key)
     if ws is None or ws.numel() < numel:
-        ws = torch.empty(numel, device=device, dtype=torch.float32)
-        _split_ws[key] = ws
+        ws = held[key] = torch.empty(numel, device=device, dtype=torch.float32)
     return ws
 
 

@@ -219,3 +219,40 @@ def test_bf16_weights_in_any_storage_order(family, order):
     _same(_grads(model, forward), want)
     with torch.no_grad():
         assert torch.isfinite(forward())
+
+
+def test_native_sequences_run_without_the_interpreter_lock():
+    """What launches several kernels or allocates from C++ lets other Python threads run meanwhile: with forced switches out
+    of the picture a second thread gets its turn only where a call gives the interpreter's lock up.  (The call is refused
+    behind that point: the allocator may give the lock up by itself.)"""
+    import sys
+    import threading
+
+    from speculators_amd import _lib
+
+    a, b = torch.zeros(64, 64, device="cuda").bfloat16(), torch.zeros(64, 32, device="cuda").bfloat16()
+    native = _lib.native()
+    gate, ran, attempts = threading.Lock(), [], 0
+    gate.acquire()
+
+    def other():
+        with gate:
+            ran.append(True)
+
+    thread = threading.Thread(target=other)
+    thread.start()
+    interval = sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(1000.0)
+        gate.release()
+        while not ran and attempts < 20000:
+            attempts += 1
+            try:
+                native.product(0, a, b, None, 1, None)
+            except ValueError:
+                pass
+        got = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+    thread.join()
+    assert got

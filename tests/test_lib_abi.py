@@ -90,3 +90,65 @@ def test_resolve_loss_config_mirrors_reference_errors():
         L.resolve_loss_config('{"zz": 1}')
     with pytest.raises(ValueError, match="must be a number"):
         L.resolve_loss_config('{"ce": "x"}')
+
+
+def test_entry_points_run_without_the_interpreter_lock():
+    """A call into the library lets other Python threads run (a launch may wait for queue space): with forced switches
+    out of the picture a second thread gets its turn only where a call gives the lock up."""
+    import sys
+    import threading
+
+    from speculators_amd import _lib
+
+    native = _lib.native()
+    gate, ran, attempts = threading.Lock(), [], 0
+    gate.acquire()
+
+    def other():
+        with gate:
+            ran.append(True)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    thread.start()
+    try:
+        sys.setswitchinterval(1000.0)
+        gate.release()  # the other thread waits for the interpreter's lock from here on
+        while not ran and attempts < 200000:
+            attempts += 1
+            try:  # (refused for its arguments: needs no GPU)
+                native.spx_rmsnorm_dweight(None, 0, 0, None, None)
+            except _lib.SpxError:
+                pass
+        got = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+    thread.join()
+    assert got
+
+
+def test_product_workspaces_belong_to_one_thread():
+    """Two threads on one stream may interleave the launches of their products: each has a buffer of its own, kept while
+    the thread lives."""
+    import threading
+    import weakref
+
+    import torch
+
+    from speculators_amd import gemm
+
+    cpu = torch.device("cpu")
+    mine = gemm._split_workspace(cpu, 64)
+    assert gemm._split_workspace(cpu, 32) is mine
+    other = []
+
+    def work():
+        ws = gemm._split_workspace(cpu, 64)
+        assert ws is gemm._split_workspace(cpu, 64)
+        other.append((ws.data_ptr() != mine.data_ptr(), weakref.ref(ws)))
+
+    thread = threading.Thread(target=work)
+    thread.start()
+    thread.join()
+    assert other[0][0] and other[0][1]() is None
+    assert gemm._split_workspace(cpu, 64) is mine
