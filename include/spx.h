@@ -337,13 +337,17 @@ int spx_ttt_attn_fwd(const void* q, int64_t q_head_stride, const void* k,
 
 /* spx_ttt_attn_fwd without a workspace argument, for callers that cannot allocate one:
  * code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has
- * no counterpart in the reference.  The forward keeps nothing in memory; shapes with
- * Hkv * D * round_up(T, 128) * 2 bytes above spx_ttt_attn_fwd_static_max_bytes() = 16 MiB are
- * rejected with status 1 (use spx_ttt_attn_fwd).  Neither this call nor anything it
- * launches allocates or frees memory.  Results are bit-identical to spx_ttt_attn_fwd.
- * The FIRST call on a device for a given head_dim raises the kernel's dynamic-LDS limit, which is
- * not allowed while a stream is being captured: make one call per device and head_dim outside
- * capture before capturing; every later call only launches kernels. */
+ * no counterpart in the reference.  The forward's only scratch, the key-contiguous copy
+ * V^T [Hkv, D, round_up(T, 128)] bf16 of calls large enough for one, lives in a static device array of
+ * spx_ttt_attn_fwd_static_max_bytes() = 16 MiB inside the library (each GPU the library runs
+ * on holds it until the process ends); shapes with Hkv * D * round_up(T, 128) * 2 bytes above
+ * that are rejected with status 1 (use spx_ttt_attn_fwd).  Neither this call nor anything it
+ * launches allocates or frees device memory.  Results are bit-identical to spx_ttt_attn_fwd.
+ * Calls may overlap in time (several streams, several host threads): those that use the array run one after the
+ * other on the device.  Calls under capture do without it, so replays may overlap with anything.
+ * The FIRST call on a device for a given head_dim does set-up work that is not allowed while a
+ * stream is being captured (it raises the kernel's dynamic-LDS limit and may look up the array's address): make one
+ * call per device and head_dim outside capture before capturing; every later call only launches kernels. */
 int64_t spx_ttt_attn_fwd_static_max_bytes(void);
 int spx_ttt_attn_fwd_static(const void* q, int64_t q_head_stride, const void* k,
                             int64_t k_head_stride, const void* v, int64_t v_head_stride,

@@ -17,6 +17,7 @@
 // dense mask or BlockMask exists anywhere.
 
 #include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -1306,9 +1307,8 @@ static DkvPlan dkv_plan(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
 // products at head_dim <= 128 and 16 us at 256 (at 800 TFLOP/s of a causal mask).  Measured, copy + kernel against
 // transposing reads: 512 rows, 32 heads of 64 16.9 / 13.4 us, 2048 of 128 57.7 / 58.3, 4096 of 128 145 / 147, 16384 rows of
 // 16 heads of 256 2485 / 3072.
-static bool fwd_tr(int64_t NQ, int64_t NKV, int Hq, int D) {
-  return 2. * (double)Hq * (double)NQ * (double)NKV * D < (D > 128 ? 16. : 60.) * 8e8;
-}
+static double fwd_us(int64_t NQ, int64_t NKV, int Hq, int D) { return 2. * Hq * (double)NQ * (double)NKV * D / 8e8; }
+static bool fwd_tr(int64_t NQ, int64_t NKV, int Hq, int D) { return fwd_us(NQ, NKV, Hq, D) < (D > 128 ? 16. : 60.); }
 static int64_t fwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
   return fwd_tr(NQ, NKV, Hq, D) ? 256 : round_up((int64_t)Hkv * D * round_up(NKV, 128) * 2, 256);
 }
@@ -1324,13 +1324,18 @@ static int64_t bwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int
 }
 
 template <int D, bool TR>
+static int fwd_lds(const char* fn) {
+  static std::atomic<uint64_t> lds_set;  // per instantiation, one bit per device
+  return ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>),
+                            FwdSmem<D, kFwdNW>::kBytes, lds_set, fn);
+}
+
+template <int D, bool TR>
 static int launch_fwd_as(AttnParams p, const uint16_t* vt, uint16_t* O, float* lse, hipStream_t st, const char* fn) {
   constexpr int BM = 32 * kFwdNSB * kFwdNW;
   const int n_qb = (p.NQ + BM - 1) / BM;
   constexpr int smem = FwdSmem<D, kFwdNW>::kBytes;
-  static std::atomic<uint64_t> lds_set;  // per instantiation, one bit per device
-  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>), smem, lds_set, fn))
-    return rc;
+  if (int rc = fwd_lds<D, TR>(fn)) return rc;
   hipLaunchKernelGGL((attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kFwdNW), smem,
                      st, p, vt, O, lse);
   return check_launch(fn);
@@ -1484,7 +1489,7 @@ static AttnParams ttt_params(const void* q, int64_t q_hs, const void* k, int64_t
   return p;
 }
 
-// workspace: null = none (spx_ttt_attn_fwd_static)
+// workspace: room for V^T, or null: transposing reads whatever the size (spx_ttt_attn_fwd_static)
 static int ttt_attn_fwd_impl(const char* fname, const void* q, int64_t q_head_stride, const void* k,
                              int64_t k_head_stride, const void* v, int64_t v_head_stride, const int32_t* row_lo,
                              int64_t T, int32_t ttt_step, int32_t Hq, int32_t Hkv, int32_t D, float scaling, void* out,
@@ -1649,9 +1654,55 @@ extern "C" int spx_span_attn_bwd(const void* q, int64_t q_head_stride, const voi
 }
 
 // ---------------------------------------------------------------- allocation-free variant
-// The forward as callers without an allocator use it.  It keeps nothing in memory; the limit is part of the entry
-// point's contract.
+// V^T of a large call lies in a device array of the library.  Transposing reads throughout need no array and take 3 - 5 %
+// longer at head_dim 128 and up to 10 % at 256: 8192 rows, 64 / 8 heads of 128 1003 us, from the copy 957; 16384 rows,
+// 16 / 2 heads of 256 2628 / 2386.  The array serves one call at a time: a call waits, on the device, for the event behind
+// the last one's kernels, whichever stream and host thread that came from.  A call under capture takes transposing reads:
+// nothing would order its replays.  The wait and the record cost 3 us, so the copy begins later here than in fwd_tr, at
+// 120 us of products (2048 rows, 16 heads of 256, 43 us: 89.5 us without the array, 92.3 with it; 4096 rows of 16 / 2
+// heads, 172 us: 187.3 / 178.5; 4096 rows, 32 heads of 128: 140.4 / 140.3).
 constexpr int64_t kStaticScratchBytes = 16ll << 20;
+constexpr double kStaticCopyUs = 120.;
+static __device__ __align__(256) unsigned char static_scratch[kStaticScratchBytes];
+
+constexpr int kMaxDevices = 64;
+struct StaticScratch {
+  std::mutex mu;
+  void* base = nullptr;       // this device's array (its name is no host pointer)
+  hipEvent_t idle = nullptr;  // behind the kernels of its last user
+};
+static StaticScratch g_static[kMaxDevices];
+
+static int hip_failed(const char* fn, const char* what, hipError_t e) {
+  last_error() = std::string(fn) + ": " + what + ": " + hipGetErrorString(e);
+  return SPX_ERR_HIP;
+}
+
+// launch(base of the array, or null: transposing reads) on the stream
+template <typename F>
+static int with_static_scratch(const char* fn, bool copies, hipStream_t st, F launch) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (copies && hipStreamIsCapturing(st, &capture) != hipSuccess) {
+    (void)hipGetLastError();  // (the legacy stream while another one is captured)
+    copies = false;
+  }
+  if (!copies || capture != hipStreamCaptureStatusNone) return launch(nullptr);
+  int dev = -1;
+  if (hipError_t e = hipGetDevice(&dev)) return hip_failed(fn, "hipGetDevice", e);
+  if (dev < 0 || dev >= kMaxDevices) return launch(nullptr);
+  StaticScratch& s = g_static[dev];
+  std::lock_guard<std::mutex> lock(s.mu);
+  if (!s.base)
+    if (hipError_t e = hipGetSymbolAddress(&s.base, HIP_SYMBOL(static_scratch))) return hip_failed(fn, "hipGetSymbolAddress", e);
+  if (!s.idle) {
+    if (hipError_t e = hipEventCreateWithFlags(&s.idle, hipEventDisableTiming)) return hip_failed(fn, "hipEventCreate", e);
+  } else if (hipError_t e = hipStreamWaitEvent(st, s.idle, 0)) {
+    return hip_failed(fn, "hipStreamWaitEvent", e);
+  }
+  const int rc = launch(s.base);
+  if (hipError_t e = hipEventRecord(s.idle, st)) return hip_failed(fn, "hipEventRecord", e);
+  return rc;
+}
 
 extern "C" int64_t spx_ttt_attn_fwd_static_max_bytes(void) { return kStaticScratchBytes; }
 
@@ -1660,12 +1711,19 @@ extern "C" int spx_ttt_attn_fwd_static(const void* q, int64_t q_head_stride, con
                                        const int32_t* row_lo, int64_t T, int32_t ttt_step,
                                        int32_t Hq, int32_t Hkv, int32_t D, float scaling, void* out,
                                        float* lse, void* stream) {
-  if (int rc = shape_checks(__func__, T, T, Hq, Hkv, D)) return rc;
+  const char* const fname = __func__;
+  if (int rc = shape_checks(fname, T, T, Hq, Hkv, D)) return rc;
   if ((int64_t)Hkv * D * round_up(T, 128) * 2 > kStaticScratchBytes)
-    return fail_arg(__func__, "Hkv * D * round_up(T, 128) * 2 bytes exceed 16 MiB, the limit of this entry point; "
-                              "use spx_ttt_attn_fwd with a caller-owned workspace");
-  return ttt_attn_fwd_impl(__func__, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq,
-                           Hkv, D, scaling, out, lse, nullptr, stream);
+    return fail_arg(fname, "Hkv * D * round_up(T, 128) * 2 bytes exceed 16 MiB, the limit of this entry point; "
+                           "use spx_ttt_attn_fwd with a caller-owned workspace");
+  const bool copies = fwd_us(T, T, Hq, D) >= kStaticCopyUs;
+  return with_static_scratch(fname, copies, reinterpret_cast<hipStream_t>(stream), [&](void* workspace) {
+    if (int rc = ttt_attn_fwd_impl(fname, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq, Hkv,
+                                   D, scaling, out, lse, workspace, stream))
+      return rc;
+    // the form that captured calls take is set up by the first call too, which is made outside capture
+    return D == 256 ? fwd_lds<256, true>(fname) : D == 128 ? fwd_lds<128, true>(fname) : fwd_lds<64, true>(fname);
+  });
 }
 
 // ================================================================ DFlash entry points

@@ -72,3 +72,76 @@ def test_static_scratch_rejects_shapes_above_its_limit():
     rc = lib.spx_ttt_attn_fwd_static(None, 0, None, 0, None, 0, None, 16384, 0, 32, 8, 128, 0.1,
                                      None, None, None)
     assert rc == 1 and b"16 MiB" in lib.spx_last_error()
+
+
+# (a call below the size from which V is copied into the array, and calls above it at each head size)
+_STATIC = [(700, 8, 2, 64, 0), (4096, 32, 8, 128, 1), (6000, 32, 4, 64, 0), (3800, 16, 4, 256, 0)]
+
+
+def _static_case(t, hq, hkv, d, step, seed):
+    from speculators_amd.attention import create_ttt_mask
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    row_lo = create_ttt_mask(torch.zeros(1, t, dtype=torch.long, device="cuda"), t).row_lo
+    q = torch.randn(1, hq, t, d, device="cuda", generator=g).bfloat16()
+    k, v = (torch.randn(1, hkv, (step + 1) * t, d, device="cuda", generator=g).bfloat16() for _ in range(2))
+    ref, _ = _run(False, q, k, v, row_lo, t, step, hq, hkv, d)
+    out = torch.empty_like(ref)
+    lse = torch.empty(hq, t, device="cuda")
+
+    def call():
+        from speculators_amd import _lib
+
+        _lib.call("spx_ttt_attn_fwd_static", q, q.stride(1), k, k.stride(1), v, v.stride(1), row_lo, t, step, hq, hkv, d,
+                  float(d ** -0.5), out, lse, _lib.stream_ptr(q.device))
+
+    return call, out, ref
+
+
+def test_static_scratch_serves_streams_and_threads_at_once():
+    """Calls that overlap in time, of several streams and host threads and with different inputs, do not see each other's
+    copy of V."""
+    import threading
+
+    cases = [[_static_case(*shape, seed=10 * i + j) for j, shape in enumerate(_STATIC)] for i in range(3)]
+    torch.cuda.synchronize()
+
+    def work(mine):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(6):
+                for call, _, _ in mine:
+                    call()
+
+    threads = [threading.Thread(target=work, args=(mine,)) for mine in cases]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    for mine in cases:
+        for _, out, ref in mine:
+            assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("shape", _STATIC)
+def test_static_scratch_is_not_held_by_a_graph(shape):
+    """Replays of a captured call next to eager calls of the same size on another stream."""
+    call, out, ref = _static_case(*shape, seed=1)
+    other, other_out, other_ref = _static_case(*shape, seed=2)
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        out.fill_(7.0)
+        other_out.fill_(7.0)
+        torch.cuda.synchronize()
+        for _ in range(3):
+            graph.replay()
+            with torch.cuda.stream(side):
+                other()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+        assert torch.equal(other_out.view(torch.int16), other_ref.view(torch.int16))
