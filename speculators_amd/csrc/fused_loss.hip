@@ -201,6 +201,14 @@ __device__ __forceinline__ void add_second(float& acc, float& ext, const float (
   }
 }
 
+// The arg-max of a row without a value above -infinity (all of it -infinity or NaN, where tail padding may have won, too) is
+// 0, as torch has it: whatever a row holds and whatever known statistics say, the indices are columns of it.
+template <typename T>
+__device__ __forceinline__ void settle(RowStats& s, const T* xrow, int64_t vocab) {
+  if ((uint32_t)s.id >= (uint32_t)vocab) s.id = 0;
+  if ((uint32_t)s.it >= (uint32_t)vocab) { s.it = 0; s.xt = load1(xrow); }
+}
+
 // one thread writes what a row leaves behind
 template <bool KNOWN>
 __device__ __forceinline__ void store_row(int64_t r, const RowStats& s, float row_loss, float lse_d, float row_extra,
@@ -377,9 +385,6 @@ __global__ __launch_bounds__(NT) void loss_fwd_kernel(
     add_chunk<OP, KNOWN>(s, x, y, base, lt2_known);
   }
 
-  // tail padding must never win an arg-max: padded values are kNegBig, and
-  // a padded index only enters when cx == kNegBig > -inf on an all-padding
-  // chunk, which cannot exist (every chunk holds at least one real element).
   __shared__ RowStats part[NT / 64];
   __shared__ float red[NT / 64];
   s = block_merge<NT / 64>(s, part);
@@ -387,10 +392,9 @@ __global__ __launch_bounds__(NT) void loss_fwd_kernel(
   const float lse_d = (s.md + fast_log2(s.zd)) * kLn2;
   const float lse_t = KNOWN ? lse_target[r]
                             : ((OP != SPX_LOSS_CE) ? (s.mt + fast_log2(s.zt)) * kLn2 : 0.f);
-  if (KNOWN) {
-    s.it = argmax_target ? argmax_target[r] : 0;
-    if (OP == SPX_LOSS_CE) s.xt = load1(xrow + s.it);
-  }
+  if (KNOWN) s.it = argmax_target ? argmax_target[r] : 0;
+  settle(s, xrow, vocab);
+  if (KNOWN && OP == SPX_LOSS_CE) s.xt = load1(xrow + s.it);
 
   float row_loss = 0.f, row_extra = 0.f;
   if (OP == SPX_LOSS_KL) {
@@ -565,10 +569,9 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
   const float lse_d = soft_x ? (s.md + fast_log2(s.zd)) * kLn2 : 0.f;
   const float lse_t = KNOWN ? lse_target[r]
                             : ((OP != SPX_LOSS_CE) ? (s.mt + fast_log2(s.zt)) * kLn2 : 0.f);
-  if (KNOWN) {
-    s.it = argmax_target[r];
-    if (OP == SPX_LOSS_CE) s.xt = (s.it >= 0 && s.it < vocab) ? load1(xrow + s.it) : 0.f;
-  }
+  if (KNOWN) s.it = argmax_target[r];
+  settle(s, xrow, vocab);
+  if (KNOWN && OP == SPX_LOSS_CE) s.xt = load1(xrow + s.it);
   if (tid == 0) {
     float row_loss;
     if (!soft_x) row_loss = 0.f;
@@ -857,6 +860,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_fwd_gather_pipe_kernel(
   s = part[0];
 #pragma unroll
   for (int w = 1; w < kLossWaves; ++w) merge(s, part[w]);
+  settle(s, xrow, vocab);
   const float lse_d = (s.md + fast_log2(s.zd)) * kLn2;
   const float lse_t = (OP != SPX_LOSS_CE) ? (s.mt + fast_log2(s.zt)) * kLn2 : 0.f;
   float row_loss;
@@ -1079,7 +1083,7 @@ __global__ __launch_bounds__(kLossThreads) void row_tokens_kernel(const int32_t*
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < kLossWaves; ++w) take(bl[w], al[w]);
-    out[n + (int64_t)blockIdx.x] = at;
+    out[n + (int64_t)blockIdx.x] = at < vocab ? at : 0;  // (no value above -infinity: see settle)
   }
 }
 

@@ -549,7 +549,7 @@ __global__ __launch_bounds__(256) void gemm_row_stats_reduce_kernel(const float*
     }
   }
   if (lse) lse[m] = (mm * kLog2e + fast_log2(z)) * kLn2;
-  if (argmax) argmax[m] = first;
+  if (argmax) argmax[m] = first == 0x7fffffff ? 0 : first;  // (no value above -infinity: 0, as torch has it)
 }
 
 // The tiles of the last round of a product cut by tail_plan: C[tile] = the sum of its parts, in their

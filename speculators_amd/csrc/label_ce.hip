@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kLossThreads) void label_ce_fwd_kernel(
     }
     loss[r] = l;
     lse_out[r] = lse;
-    if (argmax_out) argmax_out[r] = s.idx;
+    if (argmax_out) argmax_out[r] = s.idx < vocab ? s.idx : 0;  // (no value above -infinity: 0, as torch has it)
   }
 }
 

@@ -569,3 +569,71 @@ def test_mask_row_map_and_step_total(rows, kind):
               before, total, a, rw[1], st)
     assert torch.equal(a[:6], b) and torch.equal(rw[0], rw[1]) and a[7].item() == 1.0
     assert a[6].item() == b[0].item() * 0.25 and abs(total.item() - (2.5 + a[6].item())) < 1e-6
+
+
+def _rows_without_a_maximum(vocab, dtype):
+    """Rows of -infinity, NaN, both, and the type's lowest value with one larger value or none; plain rows between them."""
+    g = torch.Generator().manual_seed(vocab)
+    x = torch.randn(9, vocab, generator=g)
+    x[0], x[2], x[4, :] = float("-inf"), float("nan"), torch.finfo(dtype).min
+    x[6, :] = torch.finfo(dtype).min
+    x[6, vocab - 1] = -2.0
+    x[8, : vocab // 2], x[8, vocab // 2:] = float("nan"), float("-inf")
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("vocab,dtype", [(50, torch.bfloat16), (1000, torch.float32), (32000, torch.bfloat16),
+                                         (33000, torch.bfloat16), (7, torch.float32)])
+def test_arg_max_outputs_are_columns_of_the_row(vocab, dtype):
+    """Rows of -infinity, NaN or the type's lowest value (a masked-out vocabulary, a draft that diverged): every arg-max is
+    a column, torch's where it is defined, and a statistic handed in that is none reads nothing outside the row."""
+    from speculators_amd import gemm
+    from speculators_amd import losses as L
+    from speculators_amd import metrics as MT
+
+    x = _rows_without_a_maximum(vocab, dtype)
+    y = x.flip(0).contiguous()
+    want_x, want_y = (t.masked_fill(t.isnan(), float("-inf")).argmax(-1) for t in (x, y))
+    xg, yg = x.cuda().unsqueeze(0), y.cuda().unsqueeze(0)
+    assert torch.equal(MT.argmax_rows(xg)[0].cpu(), want_x)
+    for op in (L.OP_KL, L.OP_CE, L.OP_RKL, L.OP_JSD, L.OP_TV):
+        rows, am_d, am_t, lse_t = L.fused_rows(op, xg, yg)
+        assert torch.equal(am_d[0].cpu().long(), want_x) and torch.equal(am_t[0].cpu().long(), want_y)
+    # cross-entropy of a target row without a maximum: the draft's value in column 0
+    rows, _, _, _ = L.fused_rows(L.OP_CE, xg[:, 1:2], yg[:, 8:9])
+    ref = torch.logsumexp(x[1].double(), -1) - x[1, 0].double()
+    assert abs(rows.item() - ref.item()) <= 1e-5 * abs(ref.item()) + 1e-5
+    # known statistics of such a row, as an earlier pass of another program may have left them
+    for bad in (0x7fffffff, vocab, -1):
+        known = (torch.zeros(9, device="cuda"), torch.full((9,), bad, device="cuda", dtype=torch.int32))
+        rows, am_d, _, _ = L.fused_rows(L.OP_CE, xg, yg, known)
+        assert torch.equal(am_d[0].cpu().long(), want_x)
+        assert abs(rows[0, 1].item() - ref.item()) <= 1e-5 * abs(ref.item()) + 1e-5
+        if dtype == torch.bfloat16 and vocab % 8 == 0 and vocab <= 32768:
+            step = L.StepPass(mask=torch.ones(9, device="cuda"), counts=torch.zeros(3, device="cuda", dtype=torch.int32),
+                              grad_in_pass=True)
+            loss, _, am_d, *_ = L._loss_forward_with_grad(L.OP_CE, xg[0], None, known, step)
+            assert torch.equal(am_d.cpu().long(), want_x)
+            assert abs(loss[1].item() - ref.item()) <= 1e-5 * abs(ref.item()) + 1e-5
+    # the head product's epilogue: a row of NaN and one of -infinity (the product of -inf and ones)
+    a = torch.ones(4, 64, device="cuda").bfloat16()
+    a[1], a[2] = float("nan"), float("-inf")
+    _, _, am = gemm.gemm_nt_stats(a, torch.ones(max(vocab, 8), 64, device="cuda").bfloat16())
+    assert am.tolist() == [0, 0, 0, 0]
+
+
+def test_arg_max_of_gathered_targets_is_a_column():
+    """The pass that reads full-vocabulary targets through the offset table, with a target row of -infinity."""
+    from speculators_amd import losses as L
+
+    vt, vd = 4096, 1024
+    x = torch.randn(5, vd, device="cuda").bfloat16()
+    full = torch.randn(5, vt, device="cuda").bfloat16()
+    full[1] = float("-inf")
+    x[3] = float("-inf")
+    d2t = torch.arange(vd, device="cuda") * 3
+    for op in (L.OP_KL, L.OP_CE):
+        step = L.StepPass(d2t=d2t, mask=None, prev=None, counts=torch.zeros(3, device="cuda", dtype=torch.int32))
+        _, _, _, _, am_d, am_t, _, _ = L.fused_loss_forward(op, x, full, None, step)
+        assert torch.equal(am_d.long(), x.argmax(-1))
+        assert torch.equal(am_t.long(), full[:, torch.arange(vd, device="cuda") * 4].argmax(-1))
