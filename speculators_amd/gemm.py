@@ -280,6 +280,10 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
     if t > rows and not fp32:
         total = gemm_tn(a, b, out.float() if accumulate else None, accumulate, torch.float32)
         return total.to(torch.bfloat16) if out is None else out.copy_(total)
+    if t == 0:  # nothing to launch: the empty sum
+        if out is None:
+            return torch.zeros(m, n, device=a.device, dtype=out_dtype)
+        return out if accumulate else out.zero_()
     for t0 in range(0, t, rows):
         out = _lib.native().product_tn(a[t0:t0 + rows], b[t0:t0 + rows], out, accumulate or t0 > 0, fp32)
     return out

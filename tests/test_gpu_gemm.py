@@ -539,3 +539,16 @@ def test_gemm_tn_in_row_bands_rounds_a_bf16_result_once(accumulate, monkeypatch)
     assert ((out.double() - want).abs() / want).max().item() <= 2 ** -8 + 1200 * 2 ** -24
     f32 = gemm.gemm_tn(a, b, out_dtype=torch.float32)
     assert ((f32.double() - a.double().t() @ b.double()).abs() / want).max().item() <= 1200 * 2 ** -24
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gemm_tn_over_no_rows_is_zero(dtype):
+    from speculators_amd import gemm
+
+    a, b = torch.empty(0, 64, device="cuda").bfloat16(), torch.empty(0, 32, device="cuda").bfloat16()
+    got = gemm.gemm_tn(a, b, out_dtype=dtype)
+    assert got.shape == (64, 32) and got.dtype == dtype and not got.any()
+    base = torch.randn(64, 32, device="cuda").to(dtype)
+    out = base.clone()
+    assert gemm.gemm_tn(a, b, out, accumulate=True) is out and torch.equal(out, base)
+    assert gemm.gemm_tn(a, b, out) is out and not out.any()
