@@ -63,6 +63,22 @@ Tensor grad_rows(const Tensor& g) {
   return x.stride(1) == 1 ? x : x.contiguous();
 }
 
+// The backward of a norm over x [rows, h], dres (may be undefined) added to dx; the partial sums of the gain's gradient go
+// to scratch (undefined: the gain does not train).
+void norm_backward(const Tensor& x, const Tensor& gain, const Tensor& dy, const Tensor& dres, const float* rstd,
+                   const Tensor& dx, const Tensor& scratch, int64_t accumulate, void* st) {
+  const int64_t rows = x.size(0), h = x.size(1), ld_dres = dres.defined() ? dres.stride(0) : 0;
+  const uint16_t* const res = dres.defined() ? in(dres) : nullptr;
+  if (scratch.defined())
+    check(spx_rmsnorm_bwd_partial(in(x), h, in(gain), in(dy), dy.stride(0), res, ld_dres, rstd, to(dx), h, floats(scratch),
+                                  accumulate, rows, h, st),
+          "spx_rmsnorm_bwd_partial");
+  else
+    check(spx_add_rmsnorm_bwd(in(x), h, in(gain), in(dy), dy.stride(0), res, ld_dres, rstd, to(dx), h, nullptr, nullptr, rows,
+                              h, st),
+          "spx_add_rmsnorm_bwd");
+}
+
 // How gemm.py routed a product (``Route`` there)
 enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul };
 struct Products {
@@ -156,11 +172,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   const Tensor dm = rows_or_new(slot_d, t, h, y);
   const Tensor dres = dy.defined() ? grad_rows(dy) : Tensor();
   if (dn.defined()) {
-    const Tensor g = grad_rows(dn);
-    check(spx_rmsnorm_bwd_partial(in(y), h, in(gain_next), in(g), g.stride(0), dres.defined() ? in(dres) : nullptr,
-                                  dres.defined() ? dres.stride(0) : 0, rstd + t, to(dm), h, floats(scratch_next),
-                                  acc_next, t, h, st),
-          "spx_rmsnorm_bwd_partial");
+    norm_backward(y, gain_next, grad_rows(dn), dres, rstd + t, dm, scratch_next, acc_next, st);
   } else {
     dm.copy_(dres);
   }
@@ -168,9 +180,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   check(spx_swiglu_rows_bwd(in(gu), 2 * f, in(gu) + f, 2 * f, in(dact), f, to(dgu), 2 * f, to(dgu) + f, 2 * f, t, f, st),
         "spx_swiglu_rows_bwd");
   const Tensor dz = product(r_gu, dgu, bgu), da = rows_or_new(slot_o, t, h, y);
-  check(spx_rmsnorm_bwd_partial(in(mid), h, in(gain_post), in(dz), h, in(dm), h, rstd, to(da), h, floats(scratch_post),
-                                acc_post, t, h, st),
-        "spx_rmsnorm_bwd_partial");
+  norm_backward(mid, gain_post, dz, dm, rstd, da, scratch_post, acc_post, st);
   return tuple_of(released, {dm, dgu, da, product(r_o, da, bo)});
   END_HANDLE_TH_ERRORS
 }

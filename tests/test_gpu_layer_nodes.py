@@ -256,3 +256,28 @@ def test_native_sequences_run_without_the_interpreter_lock():
         sys.setswitchinterval(interval)
     thread.join()
     assert got
+
+
+@pytest.mark.parametrize("family,frozen", [(f, n) for f in FAMILIES for n in (
+    "norm", "post_attention_layernorm", "input_layernorm", "hidden_norm" if f.startswith("eagle3") else "q_norm")])
+def test_gains_that_do_not_train(family, frozen, monkeypatch):
+    """Frozen norms (all, or one of a layer's): no gradient for them, every other gradient that of the layer put together
+    from its parts."""
+    from speculators_amd import dflash, eagle3, mtp
+
+    results = []
+    for parts in (False, True):
+        model, _, forward = _family(family)
+        names = [n for n, p in model.named_parameters() if frozen in n and p.requires_grad]
+        assert names
+        for n in names:
+            model.get_parameter(n).requires_grad_(False)
+        if parts:
+            for cls in (eagle3.DecoderLayer, dflash.DFlashDecoderLayer, mtp.MTPLayer):
+                monkeypatch.setattr(cls, "_step", lambda self, *a: None)
+        results.append(_grads(model, forward))
+    (loss, grads), (want_loss, want) = results
+    assert abs(loss.item() - want_loss.item()) <= 2e-3 * abs(want_loss.item())
+    assert grads.keys() == want.keys() and not any(frozen in n for n in grads) and len(want) >= 5
+    for n, w in want.items():
+        assert (grads[n].float() - w.float()).abs().max() <= 2e-2 * w.float().abs().max() + 1e-6, n
