@@ -316,6 +316,8 @@ class BatchPacker:
                     hs_seg.append((None, dst, hs.data_offset("hidden_states"), n, fd))
                     if hs.entries["token_ids"].dtype == torch.int64:
                         ids_seg.append((None, ids0 + 8 * at, hs.data_offset("token_ids"), 8 * keep, fd))
+                    elif keep == hs.seq_len:
+                        raise ValueError(f"{hs.path}: token_ids must be int64, not {hs.entries['token_ids'].dtype}")
                     else:
                         ids = torch.empty(hs.seq_len, dtype=hs.entries["token_ids"].dtype)
                         hs.read_into("token_ids", ids)

@@ -195,6 +195,18 @@ def test_files_whose_header_or_length_is_wrong_are_refused(tmp_path, case):
     _check(packer([raw]), _want([raw], packer.max_len, 64, 3, "eagle3"))
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.float32, torch.uint8])
+def test_a_file_whose_ids_are_not_int64_is_refused(tmp_path, dtype):
+    from speculators_amd.data import BatchPacker, HiddenStatesFile
+
+    raw = _raw(10, 3, 64, torch.Generator().manual_seed(1), torch.bfloat16)
+    save_file({"hidden_states": raw["hidden_states"], "token_ids": raw["token_ids"].to(dtype)}, tmp_path / "a.safetensors")
+    packer = BatchPacker(32, 64, 3)
+    with pytest.raises(ValueError, match="token_ids"):
+        packer([{"hidden_states": HiddenStatesFile(tmp_path / "a.safetensors"), "loss_mask": raw["loss_mask"]}])
+    _check(packer([raw]), _want([raw], 32, 64, 3, "eagle3"))
+
+
 def test_loader_hands_worker_errors_to_the_caller(tmp_path):
     from speculators_amd.data import BatchPacker, PackedBatchLoader
 
