@@ -368,8 +368,9 @@ class Eagle3DraftModel(nn.Module):
         hidden = self._linear(x, self.fc.weight)
 
         # the ids of step j are the given ones shifted by j, zeros behind them: windows of one buffer
-        ids = torch.zeros(1, t + ttt_steps, device=device, dtype=input_ids.dtype)
-        ids[:, :t].copy_(input_ids.detach())
+        if input_ids.shape != (1, t):
+            raise ValueError(f"input_ids must be {(1, t)}, got {tuple(input_ids.shape)}")
+        ids = F.pad(input_ids.detach(), (0, ttt_steps))
         return_loss = verifier_last_hidden_states is not None or verifier_logits is not None
         if return_loss:
             with torch.no_grad():

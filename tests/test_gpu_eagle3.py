@@ -667,3 +667,13 @@ def test_cross_entropy_loss_never_materialises_the_verifier_logits(monkeypatch):
     for k in range(3):
         assert got[2][f"full_acc_{k}_total"].item() == rm[f"full_acc_{k}_total"].item()
         assert got[2][f"cond_acc_{k}_total"].item() == rm[f"cond_acc_{k}_total"].item()
+
+
+def test_input_ids_of_another_length_or_device_are_refused():
+    shape = _shape()
+    model = _make(shape, {k: v.bfloat16() for k, v in OE.random_weights(shape, seed=1, std=0.05).items()})
+    hs, ids, doc, mask, pos, vl = _batch(shape, 40, 2, [40])
+    rest = (doc.cuda(), mask.cuda(), pos.cuda(), vl.bfloat16().cuda())
+    for bad in (ids, ids.cuda()[:, :1], ids.cuda()[:, :39], torch.cat([ids, ids], 1).cuda()):
+        with pytest.raises((RuntimeError, ValueError)):
+            model(hs.bfloat16().cuda(), bad, *rest, ttt_steps=2)
