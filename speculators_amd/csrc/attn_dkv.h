@@ -237,7 +237,7 @@ __device__ __forceinline__ void dkv_consume(const AttnParams& p, const DkvJob& j
     if (j < LPW) {
       const bool is_do = 4 * j >= NLQ;  // (NLQ is a multiple of four)
       load_to_lds16<0>(is_do ? dres : qres, job.lds + buf * C::kTile + cw * 1024 + j * 4096,
-                       ld_off[j < LPW ? j : 0] + mq * (is_do ? p.Hq * C::RB : C::RB), 0);
+                       (int)((uint32_t)ld_off[j < LPW ? j : 0] + (uint32_t)mq * (uint32_t)(is_do ? p.Hq * C::RB : C::RB)), 0);
     } else {
       const uint32_t s = job.lds + C::kOffSmall + (cw == 3 ? C::kSets * C::kSmall : set * C::kSmall + cw * 256);
       load_to_lds4(sres, s, sm_off + mq * 4, 0);

@@ -1409,8 +1409,9 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
                        st, p, dOp, lse, delta, dQp, dq_hs);
   }
 
-  if ((int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31)) {
-    last_error() = std::string(fn) + ": queries must span less than 2 GiB";
+  // (byte offsets of dO's rows are 32 bits, without a sign; the rows that fill the last tile count)
+  if (D > 128 ? (int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31) : ((int64_t)p.NQ + 64) * p.Hq * D * 2 >= (1ll << 32)) {
+    last_error() = std::string(fn) + ": queries must span less than " + (D > 128 ? "2" : "4") + " GiB";
     return SPX_ERR_ARG;
   }
   static std::atomic<uint64_t> dkv_lds_set;  // per head_dim instantiation, one bit per device
