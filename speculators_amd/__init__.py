@@ -2,8 +2,8 @@
 backward) behind the plug-in points of vllm-project/speculators.
 
 The compute lives in ``libspx_hip.so`` (hand-written gfx950 HIP kernels behind
-a C ABI, declared in ``include/spx.h``); this package is the host side: ctypes
-bindings, autograd wrappers, and mirrors of the reference's attention-function
+a C ABI, declared in ``include/spx.h``); this package is the host side: the
+binding (a native module), autograd nodes, and mirrors of the reference's attention-function
 and loss-function registries and of its draft-model ``forward`` API.
 """
 

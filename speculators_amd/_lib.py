@@ -1,4 +1,5 @@
-"""ctypes binding of ``libspx_hip.so``.
+"""Binding of ``libspx_hip.so``: the native module ``_spx_native`` (``csrc/binding.cpp``) for the calls of this
+package, ctypes signatures of the same entry points for programs that use the C ABI directly.
 
 There is no CPU or PyTorch fallback: if the library is not built, or a call is
 made with tensors that are not on a HIP device, the call raises.

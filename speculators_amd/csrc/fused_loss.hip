@@ -123,61 +123,61 @@ __device__ __forceinline__ void load8_gather(const T* full, const int64_t* __res
 template <int OP, bool KNOWN>
 __device__ __forceinline__ void add_chunk(RowStats& s, const float (&x)[8], const float (&y)[8], int64_t base,
                                           float lt2_known) {
-      float cx = x[0], cy = y[0];
-  #pragma unroll
-      for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
-      if (!KNOWN) {
-  #pragma unroll
-        for (int i = 1; i < 8; ++i) cy = fmaxf(cy, y[i]);
-      }
-      if (cx > s.bd) {  // strict: an earlier chunk of this thread keeps a tie
-        int k = 7;
-  #pragma unroll
-        for (int i = 6; i >= 0; --i) k = (x[i] == cx) ? i : k;
-        s.bd = cx; s.id = (int)base + k;
-      }
-      if (!KNOWN && cy > s.bt) {
-        int k = 7;
-        float xv = x[7];
-  #pragma unroll
-        for (int i = 6; i >= 0; --i) {
-          const bool hit = y[i] == cy;
-          k = hit ? i : k;
-          xv = hit ? x[i] : xv;
-        }
-        s.bt = cy; s.it = (int)base + k; s.xt = xv;
-      }
-      {
-        const float cxs = cx * kLog2e;
-        float mn = s.md, z = s.zd;
-        if (cxs > mn) {  // the running max moves rarely once a few chunks have been seen
-          z *= fast_exp2(mn - cxs);
-          mn = cxs;
-        }
-  #pragma unroll
-        for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -mn));
-        s.zd = z; s.md = mn;
-      }
-      if (KNOWN && OP != SPX_LOSS_CE) {
-        float a = s.at;
-  #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float pr = fast_exp2(fmaf(y[i], kLog2e, -lt2_known));  // the target probability
-          a = fmaf(pr, y[i] - x[i], a);
-        }
-        s.at = a;
-      } else if (OP != SPX_LOSS_CE) {
-        float mn = fmaxf(s.mt, cy * kLog2e);
-        float rs = fast_exp2(s.mt - mn);
-        float z = s.zt * rs, a = s.at * rs;
-  #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float e = fast_exp2(fmaf(y[i], kLog2e, -mn));
-          z += e;
-          if (OP == SPX_LOSS_KL) a = fmaf(e, y[i] - x[i], a);
-        }
-        s.zt = z; s.at = a; s.mt = mn;
-      }
+  float cx = x[0], cy = y[0];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
+  if (!KNOWN) {
+#pragma unroll
+    for (int i = 1; i < 8; ++i) cy = fmaxf(cy, y[i]);
+  }
+  if (cx > s.bd) {  // strict: an earlier chunk of this thread keeps a tie
+    int k = 7;
+#pragma unroll
+    for (int i = 6; i >= 0; --i) k = (x[i] == cx) ? i : k;
+    s.bd = cx; s.id = (int)base + k;
+  }
+  if (!KNOWN && cy > s.bt) {
+    int k = 7;
+    float xv = x[7];
+#pragma unroll
+    for (int i = 6; i >= 0; --i) {
+      const bool hit = y[i] == cy;
+      k = hit ? i : k;
+      xv = hit ? x[i] : xv;
+    }
+    s.bt = cy; s.it = (int)base + k; s.xt = xv;
+  }
+  {
+    const float cxs = cx * kLog2e;
+    float mn = s.md, z = s.zd;
+    if (cxs > mn) {  // the running max moves rarely once a few chunks have been seen
+      z *= fast_exp2(mn - cxs);
+      mn = cxs;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -mn));
+    s.zd = z; s.md = mn;
+  }
+  if (KNOWN && OP != SPX_LOSS_CE) {
+    float a = s.at;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float pr = fast_exp2(fmaf(y[i], kLog2e, -lt2_known));  // the target probability
+      a = fmaf(pr, y[i] - x[i], a);
+    }
+    s.at = a;
+  } else if (OP != SPX_LOSS_CE) {
+    float mn = fmaxf(s.mt, cy * kLog2e);
+    float rs = fast_exp2(s.mt - mn);
+    float z = s.zt * rs, a = s.at * rs;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float e = fast_exp2(fmaf(y[i], kLog2e, -mn));
+      z += e;
+      if (OP == SPX_LOSS_KL) a = fmaf(e, y[i] - x[i], a);
+    }
+    s.zt = z; s.at = a; s.mt = mn;
+  }
 }
 
 // what the second pass over a row adds: rkl, jsd, tv
@@ -236,10 +236,6 @@ __device__ __forceinline__ void store_row(int64_t r, const RowStats& s, float ro
 }
 
 // ---- forward ---------------------------------------------------------------
-// KNOWN: lse_target / argmax_target are INPUTS (the target row's statistics from an
-// earlier pass over the same row); the target max / sum / arg-max tracking is skipped and
-// the cross-entropy reduction does not read the target row at all.
-// GATHER: the target row is read through the d2t offset table (see StepArgs).
 // eight elements as they come from memory
 template <typename T>
 struct RawChunk;
@@ -269,6 +265,11 @@ struct RawChunk<float> {
 };
 
 constexpr int gather_stage_bytes(int threads) { return threads * 128; }
+
+// KNOWN: lse_target / argmax_target are INPUTS (the target row's statistics from an
+// earlier pass over the same row); the target max / sum / arg-max tracking is skipped and
+// the cross-entropy reduction does not read the target row at all.
+// GATHER: the target row is read through the d2t offset table (see StepArgs).
 // NT: threads per row.  A call of few rows leaves compute units idle with 256 (see fwd_threads).
 template <typename T, int OP, bool VEC, bool KNOWN, bool GATHER, int NT>
 __global__ __launch_bounds__(NT) void loss_fwd_kernel(

@@ -122,7 +122,7 @@ struct Params {
   int tiles_m, tiles_n;
   int parts;                    // the contraction is cut into this many parts (> 1: fp32 partials in part_ws)
   float* part_ws;               // [parts][M][N]
-  const int32_t* tile_tab;      // grouped NT / NN: (group, first row) per tile row, see gemm_group_tiles_kernel
+  const int32_t* tile_tab;      // grouped NT / NN: (group, first row) per tile row, see group_tiles_kernel
   const int32_t* group_off;     // grouped: group boundaries
   const int32_t* m_live;        // how many leading rows of A count (device; null: all M)
   int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)

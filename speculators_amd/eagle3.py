@@ -11,7 +11,8 @@ and its state-dict names (models/eagle3/core.py:31-42), so a checkpoint of the
 reference loads with ``load_state_dict``.  The attention of every TTT step
 runs on the HIP TTT kernel, fc / lm_head / verifier head on the MFMA GEMM, the
 per-step loss, arg-maxes and acceptance counts on the fused vocabulary loss.
-The decoder-internal projections use PyTorch's (hipBLASLt) matmul.
+A decoder layer runs as one autograd node (``layer.LayerStep``); its large forward
+projections use PyTorch's (hipBLASLt) matmul where that is faster (``gemm.DECODER_GEMM``).
 """
 
 from __future__ import annotations

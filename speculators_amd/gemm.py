@@ -1,8 +1,8 @@
 """bf16 Linear products on the MFMA GEMM kernel.
 
 ``linear(x, weight)`` is ``torch.nn.functional.linear`` without bias
-(``x @ weight.T``) for bf16 tensors.  The backward computes the input gradient
-with the same NT kernel against a transposed copy of the weight
+(``x @ weight.T``) for bf16 tensors.  The backward computes the input gradient on the weight
+as it lies (NN form), or with the NT kernel against a transposed copy of it
 (``weight_t``, ``[K, N]`` contiguous) -- kept by the caller for frozen weights
 such as ``lm_head`` (model.py:70-71) so it is made once.  The weight gradient is the
 transposed-operand product ``gemm_tn``.
@@ -323,13 +323,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, weight_t: torch.Tensor | None 
 
 
 # Which GEMM runs the decoder-layer projections (q/k/v, o, gate/up, down and their input
-# gradients): "hipblaslt" = PyTorch's matmul (the library GEMM), "spx" = this library's MFMA kernel
-# (the input gradients then run against the transposed copy of the staged weight), "mixed" = each
-# where it is faster on these shapes: the forward products on hipBLASLt (6 - 12 % ahead there) except
-# those whose tile count leaves the last round of workgroups mostly idle, which this library's kernel
-# cuts along the contraction (the merged q/k/v projection: 10 % ahead of the library), the input
-# gradients on this library's kernel (8 - 20 % ahead of the library's NN product).  The fc /
-# lm_head / verifier-head products and every weight gradient always run on this library's kernels.
+# gradients): "hipblaslt" = PyTorch's matmul (the library GEMM), "spx" = this library's MFMA kernels, "mixed" =
+# each where it is faster: the forward products as ``_own_forward`` says, the input gradients on this library's
+# kernels (``input_gradient``: on the weight as it lies, or on its transposed copy).  The fc / lm_head /
+# verifier-head products and every weight gradient always run on this library's kernels.
 DECODER_GEMM = os.environ.get("SPX_DECODER_GEMM", "mixed")
 if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
     raise ValueError(f"SPX_DECODER_GEMM must be 'hipblaslt', 'spx' or 'mixed', got {DECODER_GEMM!r}")
@@ -357,8 +354,7 @@ def _project(x2: torch.Tensor, staged) -> torch.Tensor:
 
 
 def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
-    """``dy2 @ staged.w``: the input gradient of a decoder-layer projection ("mixed": this one on the
-    library's kernels, the forward product on hipBLASLt)."""
+    """``dy2 @ staged.w``: the input gradient of a decoder-layer projection."""
     # (the kernel contracts in chunks of 8: a projection a few columns wide -- a gate of width 1 --
     # stays with the library)
     if DECODER_GEMM != "hipblaslt" and dy2.shape[1] % 8 == 0 and dy2.stride(0) % 8 == 0 and dy2.stride(1) == 1:
