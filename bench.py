@@ -45,7 +45,7 @@ TRAFFIC_ROWS = {
 # The attention kernels are listed per timed call in lines that start with "[attn_step<k>]" or
 # "[attn_step<k>_w<window>]": a forward call is the V^T transpose + attn_fwd_kernel, a backward call every
 # other kernel of the section (one launch of each per call); their sums are the keys "<section>_fwd|_bwd"
-ATTN_FWD_KERNELS = ("attn_fwd_kernel", "transpose_bf16_kernel<false>")
+ATTN_FWD_KERNELS = ("attn_fwd_kernel", "transpose_bf16_kernel")
 
 
 def load_measured_traffic(path=TRAFFIC_SUMMARY):

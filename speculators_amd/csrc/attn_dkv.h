@@ -9,9 +9,9 @@
 //     half is a key half at head_dim <= 128, a half of the dims at 256) and adds dO^T P resp. Q'^T dS from the slot.
 // v_mfma_f32_16x16x32_bf16 reads a 1 KB A fragment (8 cycles of LDS) for 16 cycles of work, so a fragment has to serve
 // several products: a producer's fragment of Q' / dO serves 4 (head_dim 64, 256: 2) blocks of 16 keys, a consumer's of
-// dO^T / Q'^T serves 4.  The matrix pipe is busy 54 % of a step at head_dim 128 (1024 of 1900 cycles, 2.04 GHz); what is
-// left is the chain barrier -> soft-max -> scores of a producer and the consumers' wait for it, LDS is at 32 %.  At
-// head_dim 64 a key block of 64 leaves room for two workgroups on a compute unit, which fill each other's gaps.
+// dO^T / Q'^T serves 4.  Over whole launches the counters read: head_dim 128, 4096 rows, matrix pipe busy 46 % at 1.95 GHz,
+// LDS 31 %, waves waiting 23 % of their cycles; head_dim 256, 32760 rows, 50 % at 2.19 GHz, 43 %, 34 %.  What is left is the
+// chain barrier -> soft-max -> scores of a producer and the consumers' wait for it.  At head_dim 64 a key block of 64 leaves room for two workgroups on a compute unit, which fill each other's gaps.
 // Measured, kernel + sum of the partial results (us), against waves split by key with two 32 x 32 score tiles each:
 // 512 rows, 32 heads of 64: 37 -> 18; 4096 rows, 32 heads of 128: 387 -> 300; 8192 rows, 64 heads of 128: 2370 -> 1915;
 // 16384 rows, 16 heads of 256 (one wave per SIMD before): 5080 -> 3900.
@@ -273,8 +273,8 @@ __device__ __forceinline__ void dkv_consume(const AttnParams& p, const DkvJob& j
     for (int kb = 0; kb < 4; ++kb)
       pb[kb] = join_bf16x4(lds_get<u32x2>(s + kb * 1024), lds_get<u32x2>(s + kb * 1024 + 512));
   };
-  // The loads of a later tile go out one by one between the matrix instructions: in a row they held the wave for
-  // 600 of a step's 1900 cycles.
+  // The loads of a later tile go out one by one between the matrix instructions: in a row they hold the
+  // wave for as long as all of them take to issue.
   auto consume = [&](uint32_t t, uint32_t next, int mq, int buf, int set) __attribute__((always_inline)) {
     SPX_DKV_PRIO_MFMA();
 #pragma unroll

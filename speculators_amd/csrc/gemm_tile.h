@@ -3,9 +3,10 @@
 //
 // Direct global -> LDS loads, STAGES slabs of 64 contraction indices deep, v_mfma_f32_16x16x32_bf16, operand
 // fragments double buffered in registers, the LDS reads of the next K step and the loads of the next free slab issued
-// between the products, one barrier per slab.  What bounds them is the way from L2 into LDS: 83 GB/s per compute unit
-// (21 TB/s over the chip; a kernel that only loads reaches 25) whatever the tile -- a slab of 128 x 128 takes 0.38 us
-// where its products need 0.26 -- so a larger tile is faster per multiply-add as long as every compute unit has one.
+// between the products, one barrier per slab.  What bounds them is the way into LDS: with one tile on every compute unit
+// and K to 16384 the tiles of 64 x 128, 128 x 128 and 256 x 128 all load at 61 - 79 GB/s per compute unit (16 - 20 TB/s over
+// the chip) -- 0.31, 0.49 and 0.78 us a slab, 870, 1100 and 1380 TFLOP/s; 256 x 256, NN: 1.50 us, 1430 TFLOP/s, the
+// products bound it -- so a larger tile is faster per multiply-add as long as every compute unit has one.
 #pragma once
 
 #include "spx_common.h"

@@ -334,9 +334,11 @@ if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
 
 def _own_forward(m: int, n: int, k: int) -> bool:
     """Whether the forward product of a decoder projection runs on this library's kernels in "mixed": where the
-    smaller tiles fill the chip in one round (level with hipBLASLt or ahead: 0.65 - 1.0 of its time up to 1024 rows,
-    0.73 - 0.94 where the contraction is cut), and where the last round of the large tiles is cut along the
-    contraction (``spx_gemm_bf16_nt_tail``; the merged q/k/v projection of the 8B shape: 322 us, library 357)."""
+    smaller tiles fill the chip in one round (0.57 - 1.07 of hipBLASLt's time for the 1B, 8B and 70B shapes at 256 to
+    8192 rows, 0.57 - 1.00 where the contraction is cut), and where the last round of the large tiles is cut along the
+    contraction (``spx_gemm_bf16_nt_tail``; the merged q/k/v projection of the 8B shape: 291 us at 4096 rows, library
+    300).  Whole rounds of the large tiles mostly take 1.01 - 1.13 of the library's time.
+    (All of them: profiles/decoder_forward_products.txt.)"""
     big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
     if not big:
         return ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128
