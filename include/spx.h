@@ -98,8 +98,8 @@ int spx_fused_vocab_loss_fwd(int op, const void* logits, int64_t ld_logits,
  *       counts[2] += was        (cond_total, counted before the update)
  *       prev_correct[r] = now   (in place, in prev_correct's own element type)
  *     Integer atomics: the result does not depend on the order in which rows finish.
- *     Needs both arg-max outputs.  spx_ttt_step_mean turns the counts and the row losses
- *     into the step's scalars.
+ *     Needs both arg-max outputs.  spx_ttt_step_total (or spx_ttt_step_mean) turns the counts and
+ *     the row losses into the step's scalars.
  * Replaces, together, the t2d row slice (model.py:161-169), loss_forward_kernel
  * (losses/fused.py:91-175), both torch.argmax calls and compute_accuracy_single_step. */
 int spx_vocab_loss_step_fwd(int op, const void* logits, int64_t ld_logits,
@@ -121,7 +121,7 @@ int spx_vocab_loss_step_fwd(int op, const void* logits, int64_t ld_logits,
  *                                softmax(logits[r]) - onehot(argmax targets[r])     (ce)
  * i.e. the gradient for a row weight of ONE: what follows is linear in the rows, so the weight
  * the reduction behind the loss gives row r is applied to the result of the input-gradient
- * product (spx_unpack_rows_scaled).  Rows mapped to -1 get no gradient row; with
+ * product (spx_unpack_rows_graded).  Rows mapped to -1 get no gradient row; with
  * reuse_target_stats their target row is not read and their loss and lse_draft are written as 0
  * (a masked row's loss enters no sum), their arg-max outputs and chain update are as for any
  * row. */
@@ -775,10 +775,9 @@ int spx_gemm_bf16_tn_grouped_multi(const void* a, int64_t lda, const void* b, in
                                    int accumulate, void* stream);
 
 /* out[b][c][r] = in[b][r][c] for `batches` bf16 matrices of R x C (multiples of 8), row strides
- * ld_in / ld_out and batch strides in elements: the transposed copies the input-gradient
- * products need of a weight stack (a product against W needs W^T in this library's NT form; the
- * reference's autograd gets it from the BLAS library's NN form).  No counterpart in the
- * reference. */
+ * ld_in / ld_out and batch strides in elements: the transposed copy an input-gradient product
+ * reads where it runs in the NT form (of few, large tiles; the NN forms -- spx_gemm_bf16_auto form 1,
+ * spx_gemm_bf16_nn_grouped -- read the weight as it lies).  No counterpart in the reference. */
 int spx_transpose_bf16(const void* in, int64_t ld_in, int64_t batch_stride_in, void* out,
                        int64_t ld_out, int64_t batch_stride_out, int64_t R, int64_t C,
                        int64_t batches, void* stream);

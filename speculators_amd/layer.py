@@ -59,7 +59,6 @@ class LayerStep:
         self.slots = (self.wqkv.x_slot(t) if self.first else None, self.wo.x_slot(t), self.wgu.x_slot(t),
                       self.wd.x_slot(t), next_staged.x_slot(t) if next_staged is not None else None)
 
-
     def constants(self):
         """What the backward reads beside activations and gains, to be saved with the node."""
         return (self.positions, self.inv_freq, self.mask.row_lo, self.wqkv.w, self.wo.w, self.wgu.w, self.wd.w)

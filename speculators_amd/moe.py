@@ -6,8 +6,9 @@ reaches by wrapping ``Qwen3NextDecoderLayer`` / ``Qwen3_5MoeDecoderLayer``
 (models/mtp/model_definitions.py:159-205).  The library walks over the experts that were hit and
 gathers each one's tokens; here the ``(token, slot)`` pairs are sorted by expert once per call and
 every product -- gate/up, down, their input gradients and their weight gradients -- is ONE grouped
-launch over all experts (``spx_gemm_bf16_nt_grouped`` / ``spx_gemm_bf16_tn_grouped``), with the
-group boundaries kept on the device: the host never learns how many tokens an expert received.
+launch over all experts (``spx_gemm_bf16_nt_grouped`` / ``_nn_grouped`` on the weights as they lie /
+``spx_gemm_bf16_tn_grouped``), with the group boundaries kept on the device: the host never learns
+how many tokens an expert received.
 """
 
 from __future__ import annotations
