@@ -7,6 +7,14 @@
 // and K to 16384 the tiles of 64 x 128, 128 x 128 and 256 x 128 all load at 61 - 79 GB/s per compute unit (16 - 20 TB/s over
 // the chip) -- 0.31, 0.49 and 0.78 us a slab, 870, 1100 and 1380 TFLOP/s; 256 x 256, NN: 1.50 us, 1430 TFLOP/s, the
 // products bound it -- so a larger tile is faster per multiply-add as long as every compute unit has one.
+//
+// STAGES = 1: one slab buffer and one register set per operand, so four workgroups of 128 x 128 (two of 128 x 256) share a
+// compute unit and one's stores, loads and products run beside another's: what a product needs whose contraction is so
+// short that a workgroup is mostly start and end.
+//
+// Results leave in whole 128-byte lines (`line_pair`), past the caches where they are large (STREAM).
+// The weight gradients of 512 experts (2.1 GB from 80 rows each, operands in the memory-side cache, back to back) leave at
+// 3.2 TB/s as 64-byte pieces, 3.3 in whole lines, 3.6 past the caches and 4.6 with both.
 #pragma once
 
 #include "spx_common.h"
@@ -22,6 +30,25 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ i16x4 read_tr16(uint32_t addr) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(uintptr_t)addr);
+}
+
+// Two 16-byte pieces of one row, 64 bytes apart in memory, held by every lane (a wave: 16 rows x 4 lanes): lanes r and
+// r ^ 8 of a group of 16 exchange one piece each, after which the wave's first store (x) covers rows 0 .. 7 and its
+// second (y) rows 8 .. 15 in whole 128-byte lines.  lo: lane % 16 < 8; a lane's column is that of piece 0 if lo, else
+// of piece 1.
+__device__ __forceinline__ void line_pair(bool lo, u32x4 v0, u32x4 v1, u32x4& x, u32x4& y) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t got = __builtin_amdgcn_update_dpp(0, lo ? v1[c] : v0[c], 0x128, 0xf, 0xf, true);  // row_ror:8
+    x[c] = lo ? v0[c] : got;
+    y[c] = lo ? got : v1[c];
+  }
+}
+// (a template argument: the compiler merges the two stores of a run-time choice into the cached one)
+template <bool STREAM>
+__device__ __forceinline__ void store_line(void* p, u32x4 v) {
+  if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+  else *reinterpret_cast<u32x4*>(p) = v;
 }
 
 template <int N>
@@ -129,8 +156,8 @@ struct Params {
   int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)
 };
 
-// OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT>
+// OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C.  STREAM: non-temporal stores (OUT 0 and 2)
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM>
 __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p) {
   constexpr int kWaves = WM * WN, kMI = TM / WM / 16, kNI = TN / WN / 16;
   using OA = Operand<TM, kWaves, AT>;
@@ -224,7 +251,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
     ld_k += kTK;
     ld_at = ld_at + kStage == lds0 + STAGES * kStage ? lds0 : ld_at + kStage;
   };
-  bf16x8 fa[2][kMI], fb[2][kNI];
+  constexpr int kSets = STAGES == 1 ? 1 : 2;
+  bf16x8 fa[kSets][kMI], fb[kSets][kNI];
   uint32_t rd = 0;  // slab buffer the reads go to
   auto read_one = [&](int set, int kk, int f) __attribute__((always_inline)) {
     if (f < kMI) fa[set][f] = OA::read(a_rd, rd, wm, f, kk, lane);
@@ -250,29 +278,67 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
       }
   };
 
-  // STAGES slab buffers (past the last slab the loads bring zeros)
+  if constexpr (STAGES == 1) {
+    auto products = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s) {
+      for (int j = 0; j < kNI; ++j)
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[j][i], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll
     for (int l = 0; l < kL; ++l) issue_one(l);
-    next_load();
-  }
-  wait_vmcnt<(STAGES - 1) * kL>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+    for (int s = 0; s < nslab; ++s) {
+      wait_vmcnt<0>();
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const bool two = K - s * kTK > 32;  // (a last slab of up to 32 indices is one K step)
+      if (two) {
 #pragma unroll
-  for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
-  for (int s = 0; s < nslab; ++s) {
-    __builtin_amdgcn_sched_barrier(0);
-    step(0, 1, false);
-    // every read of slab s has returned; after the barrier for every wave (its buffer is free) and slab s + 1 has
-    // landed for everybody
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kL) : "memory");
+        for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
+        products();
+      }
+      const int kk = two ? 1 : 0;
+#pragma unroll
+      for (int f = 0; f < kMI + kNI; ++f) read_one(0, kk, f);
+      if (s + 1 < nslab) {
+        // every wave has read its fragments: the buffer is free
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        ld_k += kTK;
+#pragma unroll
+        for (int l = 0; l < kL; ++l) issue_one(l);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      products();
+    }
+  } else {
+    // STAGES slab buffers (past the last slab the loads bring zeros)
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+      for (int l = 0; l < kL; ++l) issue_one(l);
+      next_load();
+    }
+    wait_vmcnt<(STAGES - 1) * kL>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    rd = rd + kStage == STAGES * kStage ? 0 : rd + kStage;
-    step(1, 0, true);
-    next_load();
+#pragma unroll
+    for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
+    for (int s = 0; s < nslab; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      step(0, 1, false);
+      // every read of slab s has returned; after the barrier for every wave (its buffer is free) and slab s + 1 has
+      // landed for everybody
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kL) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      rd = rd + kStage == STAGES * kStage ? 0 : rd + kStage;
+      step(1, 0, true);
+      next_load();
+    }
   }
   wait_vmcnt<0>();
 
@@ -295,6 +361,30 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   if constexpr (OUT >= 2) {
     float* const Cf = reinterpret_cast<float*>(C);
     const bool fast = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(Cf) & 15) == 0);
+    if (OUT == 2 && fast) {
+      const bool lo = r16 < 8;
+#pragma unroll
+      for (int i = 0; i < kMI; ++i)
+#pragma unroll
+        for (int j = 0; j < kNI; j += 2) {
+          u32x4 x, y;
+          line_pair(lo, __builtin_bit_cast(u32x4, acc[j][i]), __builtin_bit_cast(u32x4, acc[j + 1][i]), x, y);
+          const int m = m0 + wm + i * 16 + (r16 & 7), n = n0 + wn + j * 16 + (lo ? 0 : 16) + 4 * q;
+          float* cp = Cf + (int64_t)m * p.ldc + n;
+          if (n + 4 <= p.N) {
+            if (m < M) store_line<STREAM>(cp, x);
+            if (m + 8 < M) store_line<STREAM>(cp + 8 * p.ldc, y);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (n + e >= p.N) continue;
+              if (m < M) cp[e] = __uint_as_float(x[e]);
+              if (m + 8 < M) cp[8 * p.ldc + e] = __uint_as_float(y[e]);
+            }
+          }
+        }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < kMI; ++i) {
       const int m = m0 + wm + i * 16 + r16;
@@ -317,6 +407,33 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   } else {
     uint16_t* const Cb = reinterpret_cast<uint16_t*>(C);
     const bool fast = (p.ldc % 8 == 0) && ((reinterpret_cast<uintptr_t>(Cb) & 15) == 0);
+    // odd groups of 16 lanes of block j <-> even groups of block j + 1: 8 consecutive columns per lane
+    auto pack8 = [](f32x4 a, f32x4 b) __attribute__((always_inline)) {
+      const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
+      u32x4 v;
+      v.x = s0[0]; v.y = s1[0]; v.z = s0[1]; v.w = s1[1];
+      return v;
+    };
+    if constexpr (OUT == 0 && kNI % 4 == 0) {
+      if (fast && p.N % 8 == 0) {
+        const bool lo = r16 < 8;
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+#pragma unroll
+          for (int j = 0; j < kNI; j += 4) {
+            u32x4 x, y;
+            line_pair(lo, pack8(acc[j][i], acc[j + 1][i]), pack8(acc[j + 2][i], acc[j + 3][i]), x, y);
+            const int m = m0 + wm + i * 16 + (r16 & 7);
+            const int n = n0 + wn + (j + (lo ? 0 : 2) + (q & 1)) * 16 + 4 * (q & 2);
+            if (n >= p.N) continue;
+            uint16_t* cp = Cb + (int64_t)m * p.ldc + n;
+            if (m < M) store_line<STREAM>(cp, x);
+            if (m + 8 < M) store_line<STREAM>(cp + 8 * p.ldc, y);
+          }
+        return;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < kMI; ++i) {
       const int m = m0 + wm + i * 16 + r16;
@@ -331,11 +448,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
             if (na + 16 + e < p.N) b[e] += bf16_bits_to_f32(Cb[(int64_t)m * p.ldc + na + 16 + e]);
           }
         }
-        // odd groups of 16 lanes of block j <-> even groups of block j + 1: 8 consecutive columns per lane
-        const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
-        const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
-        u32x4 v;
-        v.x = s0[0]; v.y = s1[0]; v.z = s0[1]; v.w = s1[1];
+        const u32x4 v = pack8(a, b);
         const int n = n0 + wn + (j + (q & 1)) * 16 + 4 * (q & 2);
         if (m >= M) continue;
         if (fast && n + 8 <= p.N) {

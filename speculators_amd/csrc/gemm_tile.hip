@@ -4,9 +4,13 @@
 // contraction.  A group of a grouped product is often neither: 512 experts x 80 rows each are 512 ragged row bands,
 // and their weight gradient contracts over 80 rows.  Measured there (4096 tokens, top 10 of 512 experts, gate/up
 // 2048 -> 1024; 2.1 GB of weights, 430 us at the rate of a copy):
-//   forward          256 x 256, 4 waves 573 us -> 128 x 256, 8 waves, 3 slabs 456 us
-//   input gradient   595 us + 786 us to transpose the weights -> 459 us on the weights as they lie (NN form)
-//   weight gradient  bf16, 4 waves 760 us -> 8 waves 698 us (1067 us with the fp32 result it replaces)
+//   forward          256 x 256, 4 waves 573 us -> 128 x 256, 8 waves, 3 slabs 498 -> whole lines past the caches 460
+//   input gradient   595 us + 786 us to transpose the weights -> 446 on the weights as they lie (NN form) -> one slab, two
+//                    workgroups a compute unit 435
+//   weight gradient  bf16, 4 waves 760 us -> 8 waves 696 (1067 us with the fp32 result it replaces) -> 128 x 128, one slab,
+//                    four workgroups a compute unit, whole lines past the caches 605 (467 with its operands in the
+//                    memory-side cache: what bounds it is waiting for them; each workgroup fetching its share of the
+//                    operands 1024 workgroups ahead made it 716)
 
 #include <algorithm>
 
@@ -52,13 +56,15 @@ __global__ __launch_bounds__(256) void group_tiles_kernel(const int32_t* __restr
   }
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT>
+constexpr int kCus = 256;
+
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM>
 static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
   constexpr int kSmem = (TM + TN) * kTK * 2 * STAGES;
   static std::atomic<uint64_t> lds_set;
-  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT>;
+  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmem, lds_set, fname)) return rc;
-  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT>),
+  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM>),
                      dim3((unsigned)(p.tiles_m * p.tiles_n * p.parts), (unsigned)groups_y), dim3(64 * WM * WN), kSmem,
                      st, p);
   return check_launch(fname);
@@ -73,7 +79,11 @@ static int64_t table_entries(int64_t rows, int64_t groups, int tm) { return (row
 template <bool BT>
 static int grouped_rows(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb,
                         int64_t b_group_stride, void* c, int64_t ldc, int64_t rows, int64_t N, int64_t K,
-                        const int32_t* group_off, int64_t groups, void* workspace, bool wide_m, hipStream_t st) {
+                        const int32_t* group_off, int64_t groups, void* workspace, hipStream_t st) {
+  // Rows a group on average: above 256 the taller tile reads the group's weights half as often (64 groups of 1024 rows,
+  // K 2048 -> N 1536, 768 -> 2048: NT 413 -> 404 us, 254 -> 240; of 4096: 1568 -> 1385, 978 -> 876; of 256, 512 groups:
+  // 1054 -> 1084, 634 -> 641; NN 220 -> 220, 457 -> 425; of 256: 550 -> 584, 1095 -> 1095).
+  const bool wide_m = rows > 256 * groups;
   const int tm = wide_m ? 256 : 128;
   const int64_t max_tiles = table_entries(rows, groups, tm), tiles_n = (N + 255) / 256;
   SPX_REQ_FN(max_tiles * tiles_n < (1ll << 31), "too many tiles");
@@ -89,8 +99,12 @@ static int grouped_rows(const char* fname, const void* a, int64_t lda, const voi
   p.M = (int)rows; p.N = (int)N; p.K = (int)K;
   p.tiles_m = (int)max_tiles; p.tiles_n = (int)tiles_n; p.parts = 1;
   p.tile_tab = tab; p.group_off = group_off; p.group_stride = b_group_stride;
-  return wide_m ? launch<256, 256, 2, 4, 2, 2, false, BT, 0>(fname, p, 1, st)
-                : launch<128, 256, 2, 4, 3, 2, false, BT, 0>(fname, p, 1, st);
+  if (wide_m) return launch<256, 256, 2, 4, 2, 2, false, BT, 0, true>(fname, p, 1, st);
+  // A short contraction is mostly start and end of a tile: two workgroups with one slab each cover them, three slabs of
+  // one workgroup do not -- where there are tiles for two (512 groups of 80 rows: K 512 -> N 2048 NT 247 -> 236 us, K 1024
+  // -> 2048 NN 430 -> 409; 64 groups of 88 rows: 34 -> 35, 57 -> 66; K 2048: 432 / 431 NT, 234 -> 245 NN)
+  if (K <= 1024 && groups * tiles_n >= 4 * kCus) return launch<128, 256, 2, 4, 1, 4, false, BT, 0, true>(fname, p, 1, st);
+  return launch<128, 256, 2, 4, 3, 2, false, BT, 0, true>(fname, p, 1, st);
 }
 
 int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t b_group_stride,
@@ -105,7 +119,19 @@ int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int
   SPX_REQ_FN((256 * lda + K) * 2 < 0x7ffffff0ll && (256 * ldb + K) * 2 < 0x7ffffff0ll,
              "256 rows of an operand must span less than 2 GiB (32-bit offsets inside a tile)");
   return grouped_rows<false>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_off, groups, workspace,
-                             false, reinterpret_cast<hipStream_t>(stream));
+                             reinterpret_cast<hipStream_t>(stream));
+}
+
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB>
+static int launch_tn_tile(const char* fname, Params p, int64_t groups, int out, hipStream_t st) {
+  p.tiles_m = (p.M + TM - 1) / TM;
+  p.tiles_n = (p.N + TN - 1) / TN;
+  switch (out) {
+    case 0: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 0, true>(fname, p, (int)groups, st);
+    case 1: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 1, false>(fname, p, (int)groups, st);
+    case 2: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 2, true>(fname, p, (int)groups, st);
+    default: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 3, false>(fname, p, (int)groups, st);
+  }
 }
 
 int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
@@ -117,15 +143,16 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
   p.C = c;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.M = (int)M; p.N = (int)N; p.K = (int)rows;
-  p.tiles_m = (int)((M + 255) / 256); p.tiles_n = (int)((N + 255) / 256); p.parts = 1;
+  p.parts = 1;
   p.group_off = group_off; p.group_stride = c_group_stride;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  switch ((out_f32 ? 2 : 0) + (accumulate ? 1 : 0)) {
-    case 0: return launch<256, 256, 2, 4, 2, 2, true, true, 0>(fname, p, (int)groups, st);
-    case 1: return launch<256, 256, 2, 4, 2, 2, true, true, 1>(fname, p, (int)groups, st);
-    case 2: return launch<256, 256, 2, 4, 2, 2, true, true, 2>(fname, p, (int)groups, st);
-    default: return launch<256, 256, 2, 4, 2, 2, true, true, 3>(fname, p, (int)groups, st);
-  }
+  const int out = (out_f32 ? 2 : 0) + (accumulate ? 1 : 0);
+  // Up to 512 rows a group the store of a tile takes longer than its products: small workgroups that overlap one
+  // another.  (1024, 2048 results; 256 x 256 with whole lines / 128 x 128: 512 groups of 10 rows 460 / 350 us, of 80
+  // 546 / 467, of 256 (1536 columns) 1428 / 1356; 64 groups of 1024 rows 439 / 440 and, 2048 x 768, 250 / 269; of 2048
+  // rows 522 / 752.)
+  return rows <= 512 * groups ? launch_tn_tile<128, 128, 2, 2, 1, 4>(fname, p, groups, out, st)
+                              : launch_tn_tile<256, 256, 2, 4, 2, 2>(fname, p, groups, out, st);
 }
 
 // ------------------------------------------------------------------------------------------ plain products
@@ -171,7 +198,7 @@ constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (no 4-wave ker
                           {256, 128, 1, 0.59f, 0.22f, 3.9f},
                           {64, 128, 2, 0.25f, 0.48f, 0.f},
                           {256, 256, 1, 1.13f, 0.33f, 4.0f}};
-constexpr int kCus = 256, kMinSlabs = 6, kMaxParts = 12, kSplitFrom = 32;  // (no cut below 32 slabs)
+constexpr int kMinSlabs = 6, kMaxParts = 12, kSplitFrom = 32;  // (no cut below 32 slabs)
 
 struct Choice {
   int tile, parts;
@@ -243,11 +270,11 @@ static int dense_check(const char* fname, int form, const void* a, int64_t lda, 
 template <bool BT>
 static int launch_dense(const char* fname, int tile, const Params& p, hipStream_t st) {
   switch (tile) {
-    case k128x128: return launch<128, 128, 2, 4, 4, 2, false, BT, 0>(fname, p, 1, st);
-    case k256x128: return launch<256, 128, 4, 2, 3, 2, false, BT, 0>(fname, p, 1, st);
-    case k64x128: return launch<64, 128, 2, 2, 3, 2, false, BT, 0>(fname, p, 1, st);
+    case k128x128: return launch<128, 128, 2, 4, 4, 2, false, BT, 0, false>(fname, p, 1, st);
+    case k256x128: return launch<256, 128, 4, 2, 3, 2, false, BT, 0, false>(fname, p, 1, st);
+    case k64x128: return launch<64, 128, 2, 2, 3, 2, false, BT, 0, false>(fname, p, 1, st);
     default:
-      if constexpr (BT) return launch<256, 256, 2, 4, 2, 2, false, true, 0>(fname, p, 1, st);
+      if constexpr (BT) return launch<256, 256, 2, 4, 2, 2, false, true, 0, false>(fname, p, 1, st);
       return fail_arg(fname, "no such tile");
   }
 }
@@ -278,11 +305,8 @@ extern "C" int spx_gemm_bf16_nn_grouped(const void* a, int64_t lda, const void* 
   SPX_REQ_FN(((uintptr_t)a | (uintptr_t)b) % 16 == 0, "a and b must be 16-byte aligned");
   SPX_REQ_FN((256 * lda + K) * 2 < 0x7ffffff0ll && (K + 4 * tile::kTK) * ldb * 2 < 0x7ffffff0ll,
              "256 rows of a and one group of b must span less than 2 GiB (32-bit offsets)");
-  // 256 rows a group on average: the taller tile reads the group's weights half as often.  16384 tokens, top 8 of 512
-  // experts of width 768 (256 rows): 1176 us with 128 rows a tile, 1183 us with 256; 320 rows 249 / 243 us; 2560
-  // rows 833 / 729 us
   return tile::grouped_rows<true>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups,
-                                  workspace, rows > 256 * groups, reinterpret_cast<hipStream_t>(stream));
+                                  workspace, reinterpret_cast<hipStream_t>(stream));
 }
 
 // whether the contraction of a product may be cut: the partials are stored in groups of four columns
