@@ -134,6 +134,18 @@ int spx_vocab_loss_step_fwd_grad(int op, const void* logits, int64_t ld_logits,
                                  int prev_kind, int32_t* counts, const int32_t* row_map,
                                  void* grad_logits, int64_t ld_grad, void* stream);
 
+/* The same row pass for a weighted sum of terms (losses/utils.py:233-266): `terms` is a set of loss ops (bit op), each
+ * with its weight in term_weights[op] (host memory, 5 elements).  loss [n][rows]: the rows of every term, unweighted, in
+ * the order of the ops; grad_logits as above, of sum_op term_weights[op] * loss_op for a row weight of ONE, summed in
+ * fp32 and rounded once.  Always reads the target rows of live rows; without reuse_target_stats it leaves the target
+ * rows' log-sum-exp and arg-max behind whatever the terms are, with it it takes both. */
+int spx_vocab_loss_terms_fwd_grad(int32_t terms, const float* term_weights, const void* logits, int64_t ld_logits,
+                                  const void* targets, int64_t ld_targets, int64_t rows, int64_t vocab, float* loss,
+                                  float* lse_draft, float* lse_target, int32_t* argmax_draft, int32_t* argmax_target,
+                                  int reuse_target_stats, const void* mask, int mask_kind, void* prev_correct,
+                                  int prev_kind, int32_t* counts, const int32_t* row_map, void* grad_logits,
+                                  int64_t ld_grad, void* stream);
+
 /* grad_logits[r, :] = g_r * dL_r/dlogits, g_r = row_grad[r] * (*scale)
  * (scale may be NULL = 1).  Rows with g_r == 0 are written as exact zeros
  * without reading the inputs.  Closed forms of losses/fused.py:11-18; replaces
@@ -278,6 +290,13 @@ int spx_ttt_step_total(const float* loss, const int32_t* argmax_draft, const int
                        const void* mask, int mask_kind, void* prev_correct, int prev_kind, int64_t rows,
                        float weight, const int32_t* counts, float factor, const float* total_in,
                        float* total_out, float* out, float* row_weight, void* stream);
+
+/* The scalars of a step whose loss has several terms, in one launch (acceptance chain done, counts as above): out has 18
+ * elements, out[0] = out[6] = sum_op term_weights[op] * mean_op, out[8 + op] = mean_op (0 for an op that is no term),
+ * out[13 + op] = 1, the others as spx_ttt_step_total; *total_out = out[6] (+ *total_in); row_weight as there. */
+int spx_ttt_step_terms(int32_t terms, const float* term_weights, const float* loss, const void* mask, int mask_kind,
+                       int64_t rows, float weight, const int32_t* counts, const float* total_in, float* total_out,
+                       float* out, float* row_weight, void* stream);
 
 /* spx_pack_row_map for a row mask of any element kind (live: not zero); zero3 (int32[3], may be NULL) is
  * cleared: the counts of the loss pass that follows. */

@@ -43,6 +43,7 @@ SIGNATURES["spx_vocab_loss_step_fwd"] = [_I, _P, _I64, _P, _I64, _P, _I64, _P, _
                                          _P, _P, _P, _I, _P, _I, _P, _I, _P, _P]
 SIGNATURES["spx_ttt_step_mean"] = [_P, _P, _I, _I64, _F, _P, _P, _P, _P]
 SIGNATURES["spx_ttt_step_total"] = [_P, _P, _P, _P, _I, _P, _I, _I64, _F, _P, _F, _P, _P, _P, _P, _P]
+SIGNATURES["spx_ttt_step_terms"] = [_I32, _P, _P, _P, _I, _I64, _F, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_map"] = [_P, _I, _I64, _P, _P, _P, _P]
 SIGNATURES["spx_row_tokens"] = [_P, _I64, _P, _I64, _I64, _I64, _I, _P, _P]
 SIGNATURES["spx_span_attn_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _F, _P, _P,
@@ -93,6 +94,8 @@ SIGNATURES["spx_unpack_rows_graded"] = [_P, _I64, _P, _P, _P, _F, _I64, _I64, _I
 SIGNATURES["spx_unpack_rows_scaled"] = [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I64, _P]
 SIGNATURES["spx_vocab_loss_step_fwd_grad"] = [_I, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _I,
                                               _P, _I, _P, _I, _P, _P, _P, _I64, _P]
+SIGNATURES["spx_vocab_loss_terms_fwd_grad"] = [_I32, _P, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _I, _P, _I, _P,
+                                               _I, _P, _P, _P, _I64, _P]
 SIGNATURES["spx_gemm_bf16_nt_tail"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P]
 SIGNATURES["spx_gemm_tail_workspace_bytes"] = []
 SIGNATURES["spx_gemm_bf16_nt_stats"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _P]

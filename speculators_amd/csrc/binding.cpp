@@ -131,6 +131,7 @@ PyMethodDef g_methods[] = {
     SPX_HOST("normed_backward", spx_layer_normed_backward)
     SPX_HOST("product_tn", spx_layer_product_tn)
     SPX_HOST("loss_step", spx_layer_loss_step)
+    SPX_HOST("loss_terms", spx_layer_loss_terms)
     SPX_HOST("cat_bf16", spx_layer_cat_bf16)
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},
     {nullptr, nullptr, 0, nullptr}};

@@ -387,6 +387,63 @@ PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The same for a loss of several terms (spx_vocab_loss_terms_fwd_grad); d2t: the targets are full-vocabulary rows, gathered
+// first by the pass that leaves their statistics behind
+PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("loss_terms", args, n, 18);
+  const int32_t terms = (int32_t)x.integer();
+  float weights[5];
+  for (float& w : weights) w = (float)x.number();
+  const Tensor &logits = x.tensor(), &targets = x.tensor();
+  const Tensor d2t = x.maybe(), known_lse = x.maybe(), known_arg = x.maybe(), &mask = x.tensor();
+  const int64_t mask_kind = x.integer();
+  const Tensor prev = x.maybe();
+  const int64_t prev_kind = x.integer();
+  const Tensor total_in = x.maybe();
+  const double weight = x.number();
+  const Tensor& out = x.tensor();
+  Unlocked released;
+  const int64_t rows = logits.size(0), vocab = logits.size(1);
+  bool known = known_lse.defined();
+  void* const st = stream_of(logits);
+  const auto i32 = logits.options().dtype(at::kInt), f32 = logits.options().dtype(at::kFloat);
+  const Tensor map = at::empty({rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({9 * rows}, f32),
+               packed = at::empty({rows, vocab}, logits.options()), total = at::empty({}, f32);
+  int32_t* const row_map = map.mutable_data_ptr<int32_t>();
+  int32_t* const am = arg.mutable_data_ptr<int32_t>();
+  int32_t* const counts = am + 2 * rows;
+  float* const s = floats(stats);  // lse_draft, lse_target, row weights, one more, up to five terms' losses
+  float* const lse_t = known ? known_lse.mutable_data_ptr<float>() : s + rows;
+  int32_t* const am_t = known ? known_arg.mutable_data_ptr<int32_t>() : am + rows;
+  check(spx_mask_row_map(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows, counts, st), "spx_mask_row_map");
+  Tensor gathered;
+  if (d2t.defined()) {
+    gathered = at::empty({rows, vocab}, logits.options());
+    check(spx_vocab_loss_step_fwd(SPX_LOSS_KL, in(logits), logits.stride(0), in(targets), targets.stride(0),
+                                  d2t.const_data_ptr<int64_t>(), targets.size(1), to(gathered), vocab, rows, vocab,
+                                  SPX_DTYPE_BF16, s + 4 * rows, s, lse_t, s + 3 * rows, am, am_t, 0, nullptr, 0, nullptr, 0,
+                                  nullptr, st),
+          "spx_vocab_loss_step_fwd");
+    known = true;
+  }
+  const Tensor& y = gathered.defined() ? gathered : targets;
+  check(spx_vocab_loss_terms_fwd_grad(terms, weights, in(logits), logits.stride(0), in(y), y.stride(0), rows, vocab,
+                                      s + 4 * rows, s, lse_t, am, am_t, known, mask.const_data_ptr(), mask_kind,
+                                      prev.defined() ? prev.mutable_data_ptr() : nullptr, prev_kind, counts, row_map,
+                                      to(packed), vocab, st),
+        "spx_vocab_loss_terms_fwd_grad");
+  check(spx_ttt_step_terms(terms, weights, s + 4 * rows, mask.const_data_ptr(), mask_kind, rows, weight, counts,
+                           total_in.defined() ? total_in.const_data_ptr<float>() : nullptr, floats(total), floats(out),
+                           s + 2 * rows, st),
+        "spx_ttt_step_terms");
+  const bool given = known_lse.defined();
+  return tuple_of(released, {total, arg.narrow(0, 0, rows), given ? known_arg : arg.narrow(0, rows, rows),
+                             given ? known_lse : stats.narrow(0, rows, rows), packed, map.narrow(0, 0, rows),
+                             map.narrow(0, rows, 1), stats.narrow(0, 2 * rows, rows), y});
+  END_HANDLE_TH_ERRORS
+}
+
 // The row-wise concatenation of one to four matrices as one bf16 matrix
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS

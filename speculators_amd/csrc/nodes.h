@@ -18,4 +18,5 @@ PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t 
 PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n);

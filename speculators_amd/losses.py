@@ -335,6 +335,18 @@ class MeanTerm:
         return total, row_weight
 
 
+def _unit_rows_backward(saved, g32, factor: float, total_rows: int):
+    """dx of the frozen head from the unit-weight logits gradient of the live rows that the row pass left behind."""
+    from .gemm import matmul_nt
+
+    packed, row_map, count, weight_t, row_weight = saved
+    dx_packed = matmul_nt(packed, weight_t, m_live=count)
+    dx = torch.empty(total_rows, dx_packed.shape[1], device=packed.device, dtype=packed.dtype)
+    _lib.call("spx_unpack_rows_graded", dx_packed, dx_packed.stride(0), row_map, row_weight, g32, factor,
+              row_map.numel(), total_rows, dx.shape[1], dx, dx.stride(0), _lib.stream_ptr(dx.device))
+    return dx
+
+
 class _HeadStepLoss(torch.autograd.Function):
     """``_HeadFusedLoss`` and the masked mean behind it as one node, which also adds the step to the loss so far:
     ``(x, total_in) -> (total, argmax_draft, argmax_target, lse_target, logits)``.
@@ -366,17 +378,11 @@ class _HeadStepLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g, _gd, _gt, _gl, _glogits):
-        from .gemm import matmul_nt
-
         if g is None:
             return (None,) * 10
         g32 = g.to(torch.float32)
         if ctx.one_pass:
-            packed, row_map, count, weight_t, row_weight = ctx.saved_tensors
-            dx_packed = matmul_nt(packed, weight_t, m_live=count)
-            dx = torch.empty(ctx.total_rows, dx_packed.shape[1], device=packed.device, dtype=packed.dtype)
-            _lib.call("spx_unpack_rows_graded", dx_packed, dx_packed.stride(0), row_map, row_weight, g32, ctx.factor,
-                      row_map.numel(), ctx.total_rows, dx.shape[1], dx, dx.stride(0), _lib.stream_ptr(dx.device))
+            dx = _unit_rows_backward(ctx.saved_tensors, g32, ctx.factor, ctx.total_rows)
         else:
             *saved, row_weight = ctx.saved_tensors
             dx = _head_rows_backward(ctx.op, saved, row_weight * (g32 * ctx.factor), ctx.total_rows)
@@ -391,6 +397,81 @@ def head_step_loss(op: int, x, weight, weight_t, targets, target_stats, n_rows: 
     t = x.shape[1]
     total, am_d, am_t, lse_t, logits = _HeadStepLoss.apply(x.reshape(t, x.shape[2]), total_in, weight, weight_t, y, op,
                                                            target_stats, n_rows, step, mean)
+    return total, am_d, am_t, lse_t, logits.view(1, t, weight.shape[0])
+
+
+# From here on a step's terms share one row pass: a chunk of eight columns for each of the row pass's 512 threads.  Three
+# steps of {"ce": 0.1, "tv": 0.9}, forward and backward, head of width 2048: 4096 rows of 32000 4.24 -> 2.93 ms, of 8192 1.30 ->
+# 0.94, of 4096 1.10 -> 0.61; 512 rows 1.1 -> 0.43 - 0.52 at any width (launches).  Shorter rows would gain as well, but
+# keep the two-node form, term by term: there its results are pinned bit for bit.
+TERMS_MIN_VOCAB = 4096
+
+
+def terms_fit(loss_config, weight, targets, d2t, mask, n_rows: int) -> bool:
+    """Whether a step's loss is a sum of terms that the one-read row pass takes (``head_terms_loss``): several terms,
+    or one that needs a second walk over the rows, on bf16 rows that fit a workgroup's registers, under a loss mask."""
+    if not HEAD_LOSS_ONE_PASS or mask is None or mask.numel() != n_rows or n_rows == 0:
+        return False
+    ops = [PRIMITIVE_OP.get(name) for name in loss_config]
+    if any(op is None or fn is not _HIP_LOSS_FN_MAP[name] for op, (name, (fn, _)) in zip(ops, loss_config.items(), strict=True)):
+        return False
+    if len(ops) == 1 and ops[0] in (OP_KL, OP_CE):
+        return False  # _HeadStepLoss
+    vocab = weight.shape[0]
+    if vocab % 8 or not TERMS_MIN_VOCAB <= vocab <= 32768 or weight.dtype != torch.bfloat16 or targets.dtype != torch.bfloat16:
+        return False
+    if d2t is not None:
+        return d2t.numel() == vocab
+    y = _rows_2d(targets)
+    return y.shape[1] == vocab and y.stride(0) % 8 == 0 and y.data_ptr() % 16 == 0
+
+
+class _HeadTermsLoss(torch.autograd.Function):
+    """``_HeadStepLoss`` for a loss of several terms: ``(x, total_in) -> (total, argmax_draft, argmax_target, lse_target,
+    logits)``.  The row pass leaves the gradient of their weighted sum behind, so the backward knows no
+    terms."""
+
+    @staticmethod
+    def forward(ctx, x2, total_in, weight, weight_t, targets, d2t, terms, known, n_rows, step, step_weight, out):
+        from .gemm import matmul_nt
+
+        logits = matmul_nt(x2, weight)
+        ctx.total_rows = logits.shape[0]
+        weights = [0.0] * 5
+        for op, w in terms:
+            weights[op] = w
+        lse_t, am_t = (None, None) if known is None else (known[0].reshape(-1), known[1].reshape(-1))
+        total, am_d, am_t, lse_t, packed, row_map, count, row_weight, rows = _lib.native().loss_terms(
+            sum(1 << op for op, _ in terms), *weights, logits[:n_rows], targets, d2t, lse_t, am_t, step.mask,
+            _lib.kind_code(step.mask), step.prev, _lib.kind_code(step.prev) if step.prev is not None else 0, total_in,
+            step_weight, out)
+        ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
+        if d2t is not None:
+            step.gathered = rows
+        ctx.mark_non_differentiable(am_d, am_t, lse_t, logits)
+        ctx.set_materialize_grads(False)
+        return total, am_d, am_t, lse_t, logits
+
+    @staticmethod
+    def backward(ctx, g, _gd, _gt, _gl, _glogits):
+        if g is None:
+            return (None,) * 12
+        dx = _unit_rows_backward(ctx.saved_tensors, g.to(torch.float32), 1.0, ctx.total_rows)
+        return (dx, g if ctx.needs_input_grad[1] else None) + (None,) * 10
+
+
+def head_terms_loss(loss_config, x, weight, weight_t, targets, d2t, target_stats, n_rows: int, step: StepPass,
+                    step_weight: float, out, total_in=None):
+    """One step's whole loss (``terms_fit``) behind the frozen head, added to ``total_in``; ``out`` (f32 ``[18]``) receives
+    the scalars of ``spx_ttt_step_terms``.  ``d2t``: ``targets`` are full-vocabulary rows, the gathered ones come back in
+    ``step.gathered``.  Returns ``(total, argmax_draft, argmax_target, lse_target, logits [1, T, Vd])``."""
+    y = _check_head(x, weight, targets, n_rows)
+    if target_stats is not None and any(s.numel() != n_rows or s.stride(-1) != 1 for s in target_stats):
+        raise ValueError("target_stats must be contiguous [rows] tensors")
+    t = x.shape[1]
+    terms = [(PRIMITIVE_OP[name], float(w)) for name, (_, w) in loss_config.items()]
+    total, am_d, am_t, lse_t, logits = _HeadTermsLoss.apply(
+        x.reshape(t, x.shape[2]), total_in, weight, weight_t, y, d2t, terms, target_stats, n_rows, step, step_weight, out)
     return total, am_d, am_t, lse_t, logits.view(1, t, weight.shape[0])
 
 

@@ -124,6 +124,62 @@ class Head:
         return self.logits
 
 
+def _flat_prev(s_prev):
+    if s_prev is None:
+        return None
+    prev1 = s_prev.reshape(-1)
+    if prev1.stride(0) != 1:
+        raise ValueError("prev_correct must be contiguous (it is updated in place)")
+    return prev1
+
+
+def _terms_step(head, targets, loss_mask, prev_correct, ttt_step, decay, loss_config, cache, return_pred, total_in,
+                return_tokens):
+    """``compute_metrics`` with the whole loss in one row pass behind the head (``losses.head_terms_loss``), or None where
+    that does not take it."""
+    n = head.x.shape[1] - ttt_step
+    gather = targets if isinstance(targets, TargetGather) and targets.compact is None and ttt_step == 0 else None
+    if isinstance(targets, TargetGather):
+        rows = targets.full if gather is not None else targets.compact
+    elif isinstance(targets, VerifierHead):
+        rows = targets.weight if targets.logits is None else targets.logits  # (its logits are bf16 rows of that width)
+        rows = rows if targets.logits is not None else rows.new_empty(0, rows.shape[0])
+    else:
+        rows = targets
+    if (head.x.shape[0] != 1 or rows is None or head.x.dtype != torch.bfloat16
+            or not L.terms_fit(loss_config, head.weight, rows, None if gather is None else gather.d2t,
+                               None if loss_mask is None else loss_mask[:, ttt_step:], n)):
+        return None
+    if gather is None and not isinstance(targets, torch.Tensor):
+        rows = targets.materialize()
+    _, s_targets, s_mask, s_prev = _step_views(head.x, rows, loss_mask, prev_correct, ttt_step)
+    out = torch.empty(18, device=head.x.device, dtype=torch.float32)
+    known = None
+    if cache is not None and cache.get("kl") is not None and gather is None:
+        known = (cache["kl"][0][ttt_step:], cache["kl"][1][ttt_step:])
+    step = L.StepPass(mask=_as_mask(s_mask), prev=_flat_prev(s_prev))
+    total, am_d, am_t, lse_t, head.logits = L.head_terms_loss(
+        loss_config, head.x, head.weight, head.weight_t, s_targets, None if gather is None else gather.d2t, known, n, step,
+        float(np.float32(decay) ** np.float32(ttt_step)), out, total_in)
+    if gather is not None:
+        gather.compact = step.gathered.view(1, n, step.gathered.shape[-1])
+    if cache is not None and known is None and ttt_step == 0:
+        cache["kl"] = (lse_t, am_t)
+    m = {f"loss_{ttt_step}_sum": out[6], f"loss_{ttt_step}_total": out[7]}
+    if len(loss_config) > 1:
+        for name in loss_config:
+            op = L.PRIMITIVE_OP[name]
+            m[f"{name}_loss_{ttt_step}_sum"] = out[8 + op]
+            m[f"{name}_loss_{ttt_step}_total"] = out[13 + op]
+    m[f"full_acc_{ttt_step}_sum"] = out[1]
+    m[f"full_acc_{ttt_step}_total"] = out[2]
+    m[f"cond_acc_{ttt_step}_sum"] = out[3]
+    m[f"cond_acc_{ttt_step}_total"] = out[4]
+    if return_tokens:
+        return total, m, row_tokens(am_d, head.logits.detach()[0, n:])
+    return (total, m, am_d) if return_pred else (total, m)
+
+
 def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
                     ttt_step_loss_decay: float, loss_config: L.LossConfig | None = None,
                     target_stats_cache: dict | None = None, return_pred: bool = False,
@@ -146,9 +202,14 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
     if isinstance(logits, Head):
         # one node for head + loss only when the whole loss is one fused reduction
         (name0, (fn0, _w0)), = list(loss_config.items())[:1]
-        single = (len(loss_config) == 1 and name0 in L.PRIMITIVE_OP and fn0 is L._HIP_LOSS_FN_MAP.get(name0)
-                  and logits.x.requires_grad and not logits.weight.requires_grad
-                  and logits.weight_t is not None)
+        frozen = logits.x.requires_grad and not logits.weight.requires_grad and logits.weight_t is not None
+        if frozen and (len(loss_config) > 1 or name0 not in ("kl_div", "ce")):
+            done = _terms_step(logits, targets, loss_mask, prev_correct, ttt_step, ttt_step_loss_decay, loss_config,
+                               target_stats_cache, return_pred, total_in, return_tokens)
+            if done is not None:
+                return done
+        single = (frozen and len(loss_config) == 1 and name0 in L.PRIMITIVE_OP
+                  and fn0 is L._HIP_LOSS_FN_MAP.get(name0))
         if single:
             head = logits
             logits = head.x[:, :, :0].detach()  # shape carrier only
@@ -182,11 +243,7 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
     weight = float(np.float32(ttt_step_loss_decay) ** np.float32(ttt_step))
 
     mask1 = None if s_mask is None else _as_mask(s_mask)
-    prev1 = None
-    if s_prev is not None:
-        prev1 = s_prev.reshape(-1)
-        if prev1.stride(0) != 1:
-            raise ValueError("prev_correct must be contiguous (it is updated in place)")
+    prev1 = _flat_prev(s_prev)
 
     multi = len(loss_config) > 1
     # (one term: its mean goes straight onto the loss so far; several: onto each other first)
