@@ -749,6 +749,16 @@ int spx_gemm_bf16_tn_f32(const void* a, int64_t lda, const void* b, int64_t ldb,
                          void* c, int64_t ldc, int64_t M, int64_t N, int64_t T,
                          int accumulate, void* stream);
 
+/* Either of the two (out_f32) on the tiles its size asks for: results of few 256 x 256 tiles run on smaller ones, small
+ * results over many rows with the contraction in parts (fp32 partials in `workspace`, added in a fixed order, with what c
+ * holds where the product accumulates, one rounding).  workspace may be NULL (never cut); spx_gemm_tn_parts says into how
+ * many parts a product is cut that has one. */
+int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T);
+int64_t spx_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t T);
+int spx_gemm_bf16_tn_auto(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
+                          int64_t N, int64_t T, int out_f32, int accumulate, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
 /* ---------------------------------------------------------------- sparse MoE block
  * The expert products of the MoE MLP of the hybrid MTP flavours (Qwen3NextSparseMoeBlock /
  * Qwen3NextExperts of the library, reached through models/mtp/model_definitions.py:159-205).

@@ -424,8 +424,8 @@ static int launch_tn(const char* fname, const void* a, int64_t lda, const void* 
   return check_launch(fname);
 }
 
-static int gemm_tn_check(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb,
-                         const void* c, int64_t ldc, int64_t M, int64_t N, int64_t T) {
+int tile::tn_check(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, const void* c,
+                   int64_t ldc, int64_t M, int64_t N, int64_t T) {
   SPX_REQ_FN(M > 0 && N > 0 && T > 0, "M, N, T must be positive");
   SPX_REQ_FN(M < (1ll << 31) && N < (1ll << 31) && T < (1ll << 31), "dimension too large");
   SPX_REQ_FN(a && b && c, "null buffer");
@@ -441,7 +441,7 @@ static int gemm_tn_check(const char* fname, const void* a, int64_t lda, const vo
 extern "C" int spx_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                                 int64_t ldc, int64_t M, int64_t N, int64_t T, int accumulate,
                                 void* stream) {
-  if (int rc = gemm_tn_check(__func__, a, lda, b, ldb, c, ldc, M, N, T)) return rc;
+  if (int rc = tile::tn_check(__func__, a, lda, b, ldb, c, ldc, M, N, T)) return rc;
   return accumulate ? launch_tn<1>(__func__, a, lda, b, ldb, c, ldc, M, N, T, stream)
                     : launch_tn<0>(__func__, a, lda, b, ldb, c, ldc, M, N, T, stream);
 }
@@ -449,7 +449,7 @@ extern "C" int spx_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64
 extern "C" int spx_gemm_bf16_tn_f32(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                                     int64_t ldc, int64_t M, int64_t N, int64_t T, int accumulate,
                                     void* stream) {
-  if (int rc = gemm_tn_check(__func__, a, lda, b, ldb, c, ldc, M, N, T)) return rc;
+  if (int rc = tile::tn_check(__func__, a, lda, b, ldb, c, ldc, M, N, T)) return rc;
   return accumulate ? launch_tn<3>(__func__, a, lda, b, ldb, c, ldc, M, N, T, stream)
                     : launch_tn<2>(__func__, a, lda, b, ldb, c, ldc, M, N, T, stream);
 }
@@ -459,7 +459,7 @@ extern "C" int spx_gemm_bf16_tn_grouped(const void* a, int64_t lda, const void* 
                                         int64_t rows, const int32_t* group_offsets, int64_t groups,
                                         int out_f32, int accumulate, void* stream) {
   const char* fname = __func__;
-  if (int rc = gemm_tn_check(fname, a, lda, b, ldb, c, ldc, M, N, rows)) return rc;
+  if (int rc = tile::tn_check(fname, a, lda, b, ldb, c, ldc, M, N, rows)) return rc;
   SPX_REQ_FN(group_offsets && groups > 0 && groups < 65536, "null group offsets or a group count outside 1 .. 65535");
   SPX_REQ_FN(c_group_stride >= (M - 1) * ldc + N, "groups of c overlap");
   SPX_REQ_FN(c_group_stride % (out_f32 ? 4 : 8) == 0, "the groups of c must be 16-byte aligned among each other");
@@ -481,7 +481,7 @@ extern "C" int spx_gemm_bf16_tn_grouped_multi(const void* a, int64_t lda, const 
                                               const int32_t* group_offsets, int64_t groups, int out_f32,
                                               int accumulate, void* stream) {
   const char* fname = __func__;
-  if (int rc = gemm_tn_check(fname, a, lda, b, ldb, c, ldc, M, N, segment_rows)) return rc;
+  if (int rc = tile::tn_check(fname, a, lda, b, ldb, c, ldc, M, N, segment_rows)) return rc;
   SPX_REQ_FN(group_offsets && groups > 0 && groups < 65536, "null group offsets or a group count outside 1 .. 65535");
   SPX_REQ_FN(segments > 0 && segments <= 64, "1 .. 64 segments");
   SPX_REQ_FN(c_group_stride >= (M - 1) * ldc + N, "groups of c overlap");

@@ -156,8 +156,10 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
 }
 
 // ------------------------------------------------------------------------------------------ plain products
-// C[m, n .. n + 7] = the sum of the parts of a product whose contraction was cut, in their order, fp32, one rounding
-__global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ C,
+// C[m, n .. n + 7] = the sum of the parts of a product whose contraction was cut, in their order, fp32, one rounding.
+// OUT as in gemm_tile_kernel.
+template <int OUT>
+__global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ ws, void* __restrict__ C,
                                                            int64_t ldc, int M_host, int N, int parts,
                                                            const int32_t* __restrict__ m_live) {
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
@@ -171,10 +173,32 @@ __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restri
     lo += *reinterpret_cast<const f32x4*>(src);
     hi += *reinterpret_cast<const f32x4*>(src + 4);
   }
-  u32x4 v;
-  v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
-  v.z = pack_bf16x2(hi[0], hi[1]); v.w = pack_bf16x2(hi[2], hi[3]);
-  *reinterpret_cast<u32x4*>(C + (int64_t)m * ldc + n) = v;
+  if constexpr (OUT >= 2) {
+    f32x4* const cp = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + (int64_t)m * ldc + n);
+    if (OUT == 3) { lo += cp[0]; hi += cp[1]; }
+    cp[0] = lo;
+    cp[1] = hi;
+  } else {
+    u32x4* const cp = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(C) + (int64_t)m * ldc + n);
+    if (OUT == 1) {
+      const u32x4 old = *cp;
+      lo += f32x4{bf16_lo(old.x), bf16_hi(old.x), bf16_lo(old.y), bf16_hi(old.y)};
+      hi += f32x4{bf16_lo(old.z), bf16_hi(old.z), bf16_lo(old.w), bf16_hi(old.w)};
+    }
+    u32x4 v;
+    v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
+    v.z = pack_bf16x2(hi[0], hi[1]); v.w = pack_bf16x2(hi[2], hi[3]);
+    *cp = v;
+  }
+}
+
+template <int OUT>
+static int launch_reduce(const char* fname, const float* ws, void* c, int64_t ldc, int64_t M, int64_t N, int parts,
+                         const int32_t* m_live, hipStream_t st) {
+  const int64_t items = M * (N / 8);
+  hipLaunchKernelGGL(parts_reduce_kernel<OUT>, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, ws, c, ldc, (int)M,
+                     (int)N, parts, m_live);
+  return check_launch(fname);
 }
 
 // The tile a product gets.  Every candidate's time is predicted and the shortest taken:
@@ -198,6 +222,18 @@ constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (no 4-wave ker
                           {256, 128, 1, 0.59f, 0.22f, 3.9f},
                           {64, 128, 2, 0.25f, 0.48f, 0.f},
                           {256, 256, 1, 1.13f, 0.33f, 4.0f}};
+// Weight gradients (contraction slow in both operands): the candidates beside the 256 x 256 kernel of gemm_bf16_tn.hip,
+// which keeps whole rounds of its tiles and is given up only for a predicted tenth.  Fitted the same way to 128 products
+// (results of 1 .. 768 large tiles, 256 .. 20000 rows, up to 12 parts; 6 - 13 % rms).  Over them the choice takes 0.52 of that
+// kernel alone and is within 2.6 % of the best candidate (geometric means; one at 1.03 of it): 2048 x 2048 over 888 rows 29
+// -> 14 us, over 1536 40 -> 21; 3072 x 2048 over 1536 41 -> 27; 2048 x 10240 over 1777 97 -> 84; 1024 x 2048 over 2665, in
+// two bands of 256 x 256 tiles and a sum before, 49 -> 19; 512 x 512 over 5000 95 -> 15.
+constexpr Config kTN[] = {{256, 256, 1, 0.97f, 0.50f, 13.9f},
+                          {128, 128, 1, 0.29f, 0.23f, 4.5f},   // 8 waves, 4 slabs
+                          {256, 128, 1, 0.50f, 0.34f, 6.8f},
+                          {64, 128, 2, 0.22f, 0.42f, 3.4f},
+                          {128, 128, 2, 0.40f, 0.57f, 4.2f}};  // 4 waves, 2 slabs: two workgroups a compute unit
+constexpr int kTnParts = 32;
 constexpr int kMinSlabs = 6, kMaxParts = 12, kSplitFrom = 32;  // (no cut below 32 slabs)
 
 struct Choice {
@@ -247,6 +283,34 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
     }
   }
   return best;
+}
+
+static Choice choose_tn(int64_t M, int64_t N, int64_t T, bool can_split) {
+  const int slabs = (int)((T + kTK - 1) / kTK);
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
+  Choice best{kBig, 1, predict(kTN[kBig], big, slabs) / 1.1f};
+  if (big % kCus == 0) return best;
+  for (int t = 1; t < 5; ++t) {
+    const Config& c = kTN[t];
+    const int64_t tiles = ((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
+    for (int parts = 1; parts <= kTnParts; ++parts) {
+      if (parts > 1 && (!can_split || slabs / parts < kMinSlabs || tiles * parts > (int64_t)kCus * c.per_cu)) break;
+      float us = predict(c, tiles * parts, (slabs + parts - 1) / parts);
+      if (parts > 1) us += reduce_us(parts * M * N);
+      if (us < best.us) best = Choice{t, parts, us};
+    }
+  }
+  return best;
+}
+
+template <int OUT>
+static int launch_tn_dense(const char* fname, int tile, const Params& p, hipStream_t st) {
+  switch (tile) {
+    case 1: return launch<128, 128, 2, 4, 4, 2, true, true, OUT, false>(fname, p, 1, st);
+    case 2: return launch<256, 128, 4, 2, 3, 2, true, true, OUT, false>(fname, p, 1, st);
+    case 3: return launch<64, 128, 2, 2, 3, 2, true, true, OUT, false>(fname, p, 1, st);
+    default: return launch<128, 128, 2, 2, 2, 2, true, true, OUT, false>(fname, p, 1, st);
+  }
 }
 
 static int dense_check(const char* fname, int form, const void* a, int64_t lda, const void* b, int64_t ldb,
@@ -362,9 +426,52 @@ extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const vo
   if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st))
     return rc;
   if (ch.parts == 1) return SPX_OK;
-  const int64_t items = M * (N / 8);
-  hipLaunchKernelGGL(tile::parts_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, p.part_ws,
-                     reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, ch.parts, m_live);
-  return check_launch(fname);
+  return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st);
+}
+
+// ------------------------------------------------------------------------------------------ weight gradients
+extern "C" int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T) {
+  if (M <= 0 || N <= 0 || T <= 0) return 1;
+  return tile::choose_tn(M, N, T, true).parts;
+}
+
+extern "C" int64_t spx_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t T) {
+  const int32_t parts = spx_gemm_tn_parts(M, N, T);
+  return parts > 1 ? (int64_t)parts * M * N * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int spx_gemm_bf16_tn_auto(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+                                     int64_t M, int64_t N, int64_t T, int out_f32, int accumulate, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  const char* fname = __func__;
+  if (int rc = tile::tn_check(fname, a, lda, b, ldb, c, ldc, M, N, T)) return rc;
+  const bool vec = ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;  // (what the pass that adds the parts stores)
+  const tile::Choice ch = tile::choose_tn(M, N, T, vec && workspace);
+  if (ch.tile == tile::kBig || (accumulate && ch.parts == 1))  // (the small tiles write results, they add to none)
+    return (out_f32 ? spx_gemm_bf16_tn_f32 : spx_gemm_bf16_tn)(a, lda, b, ldb, c, ldc, M, N, T, accumulate, stream);
+  SPX_REQ_FN(ch.parts == 1 || (workspace_bytes >= (int64_t)ch.parts * M * N * (int64_t)sizeof(float) &&
+                               ((uintptr_t)workspace) % 16 == 0),
+             "workspace too small or unaligned");
+  const tile::Config& cfg = tile::kTN[ch.tile];
+  tile::Params p{};
+  p.A = reinterpret_cast<const uint16_t*>(a);
+  p.B = reinterpret_cast<const uint16_t*>(b);
+  p.C = c;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.M = (int)M; p.N = (int)N; p.K = (int)T;
+  const int64_t tiles_m = (M + cfg.tm - 1) / cfg.tm, tiles_n = (N + cfg.tn - 1) / cfg.tn;
+  SPX_REQ_FN(tiles_m * tiles_n * ch.parts < (1ll << 31), "too many tiles");
+  p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n; p.parts = ch.parts;
+  p.part_ws = reinterpret_cast<float*>(workspace);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (int rc = out_f32 ? tile::launch_tn_dense<2>(fname, ch.tile, p, st) : tile::launch_tn_dense<0>(fname, ch.tile, p, st))
+    return rc;
+  if (ch.parts == 1) return SPX_OK;
+  switch ((out_f32 ? 2 : 0) + (accumulate ? 1 : 0)) {
+    case 0: return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, nullptr, st);
+    case 1: return tile::launch_reduce<1>(fname, p.part_ws, c, ldc, M, N, ch.parts, nullptr, st);
+    case 2: return tile::launch_reduce<2>(fname, p.part_ws, c, ldc, M, N, ch.parts, nullptr, st);
+    default: return tile::launch_reduce<3>(fname, p.part_ws, c, ldc, M, N, ch.parts, nullptr, st);
+  }
 }
 #undef SPX_REQ_FN

@@ -321,19 +321,21 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
   END_HANDLE_TH_ERRORS
 }
 
-// The weight gradient a^T b: (a [T, M], b [T, N], out or None, accumulate, fp32) -> [M, N]
+// The weight gradient a^T b: (a [T, M], b [T, N], out or None, accumulate, fp32, workspace or None) -> [M, N]
 PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Args x("product_tn", args, n, 5);
+  Args x("product_tn", args, n, 6);
   const Tensor &a = x.tensor(), &b = x.tensor();
   Tensor out = x.maybe();
   const int64_t accumulate = x.integer(), f32 = x.integer();
+  const Tensor ws = x.maybe();
   Unlocked released;
   const int64_t t = a.size(0), m = a.size(1), cols = b.size(1);
   if (!out.defined()) out = at::empty({m, cols}, a.options().dtype(f32 ? at::kFloat : at::kBFloat16));
-  check((f32 ? spx_gemm_bf16_tn_f32 : spx_gemm_bf16_tn)(in(a), a.stride(0), in(b), b.stride(0), out.mutable_data_ptr(),
-                                                        out.stride(0), m, cols, t, accumulate, stream_of(a)),
-        "spx_gemm_bf16_tn");
+  check(spx_gemm_bf16_tn_auto(in(a), a.stride(0), in(b), b.stride(0), out.mutable_data_ptr(), out.stride(0), m, cols, t, f32,
+                              accumulate, ws.defined() ? ws.mutable_data_ptr() : nullptr,
+                              ws.defined() ? (int64_t)ws.nbytes() : 0, stream_of(a)),
+        "spx_gemm_bf16_tn_auto");
   return wrapped(released, out);
   END_HANDLE_TH_ERRORS
 }

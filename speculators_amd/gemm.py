@@ -211,25 +211,10 @@ def gemm_nt_stats(a: torch.Tensor, b: torch.Tensor, store: bool = True, want_arg
 
 
 
+@functools.lru_cache(maxsize=4096)
 def _split_bands(t: int, m: int, n: int) -> int:
-    """How many row bands the contraction of a ``[t, m]^T [t, n]`` product is cut into: enough to
-    give every compute unit a workgroup, every band at least 1024 rows long; 1 = no split."""
-    tiles = -(-m // 256) * -(-n // 256)
-    if tiles * 2 > _CUS or t < 2048:
-        return 1
-    return max(1, min(_CUS // tiles, t // 1024))
-
-
-_band_cache: dict = {}
-
-
-def _band_offsets(t: int, step: int, bands: int, device) -> torch.Tensor:
-    key = (t, step, bands, str(device))
-    off = _band_cache.get(key)
-    if off is None:
-        off = torch.tensor([min(i * step, t) for i in range(bands + 1)], dtype=torch.int32, device=device)
-        _band_cache[key] = off
-    return off
+    """How many parts the contraction of a ``[t, m]^T [t, n]`` product is cut into (``spx_gemm_bf16_tn_auto``)."""
+    return _lib.load().spx_gemm_tn_parts(m, n, t)
 
 
 def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
@@ -254,25 +239,7 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
             raise ValueError("out_dtype must be bfloat16 or float32")
     elif out.shape != (m, n) or out.dtype not in (torch.bfloat16, torch.float32) or out.stride(1) != 1:
         raise ValueError(f"out must be a bf16 or fp32 [{m}, {n}] tensor with unit column stride")
-    # A small result with a long contraction leaves most of the chip idle (one workgroup per
-    # 256 x 256 tile of the result): the contraction is then cut into row bands, every band's
-    # product goes to an fp32 partial of its own (the grouped kernel with the bands as groups) and
-    # the partials are summed in a fixed order
     fp32 = (out_dtype if out is None else out.dtype) == torch.float32
-    bands = _split_bands(t, m, n)
-    if bands > 1 and max(a.stride(0), b.stride(0)) * 2 * (t + 256) < _MAX_SPAN:
-        step = -(-t // bands)
-        off = _band_offsets(t, step, bands, a.device)
-        part = torch.empty(bands, m, n, device=a.device, dtype=torch.float32)
-        _lib.call("spx_gemm_bf16_tn_grouped", a, a.stride(0), b, b.stride(0), part,
-                  n, m * n, m, n, t, off, bands, 1, 0, _lib.stream_ptr(a.device))
-        total = part.sum(0)
-        if out is None:
-            return total if fp32 else total.to(torch.bfloat16)
-        if accumulate:
-            total += out  # in fp32: what the result holds is added before the one rounding
-        out.copy_(total)
-        return out
     # 32-bit byte offsets inside the kernel: a contraction that spans 2 GiB or more of an
     # operand is fed in bands of rows, every band after the first added to the result.  A bf16 result of several
     # bands is formed in fp32 and rounded once, like that of one
@@ -285,7 +252,10 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
             return torch.zeros(m, n, device=a.device, dtype=out_dtype)
         return out if accumulate else out.zero_()
     for t0 in range(0, t, rows):
-        out = _lib.native().product_tn(a[t0:t0 + rows], b[t0:t0 + rows], out, accumulate or t0 > 0, fp32)
+        # a small result with a long contraction: fp32 partials of its parts, summed in a fixed order
+        parts = _split_bands(min(rows, t - t0), m, n)
+        ws = _split_workspace(a.device, parts * m * n) if parts > 1 else None
+        out = _lib.native().product_tn(a[t0:t0 + rows], b[t0:t0 + rows], out, accumulate or t0 > 0, fp32, ws)
     return out
 
 
