@@ -793,68 +793,35 @@ __device__ __forceinline__ void st_bf16s(uint16_t* p, const float (&v)[EPL]) {
   }
 }
 
-// What the backward kernels read next to the operands, in one launch (five small ones took 4 us each whatever their
-// size; 512 rows of 32 heads of 64: 18 -> 6 us).  Sixteen lanes per (head, row), D / 16 consecutive elements each:
-//   qs[h][i]   bf16(q * scale * log2 e), row-major;
-//   delta      dO . O of the row (summed with DPP moves), [Hq][NQ];
-//   neg        -lse and -delta in rows of NQp (zero in the padding): C operands of the dK / dV score products;
-// and in the last blocks, one wave per 64-row query tile, the interval ends of its rows and their extremes:
-//   rows[4][NQp]  a1, b1, T + a2, T + b2 as the kernels compare them (empty where a class is absent or the row is padding)
-//   tb[tile][8]   [a1min, a1max, b1min, b1max, a2min, a2max, b2min, b2max]
-template <int D>
-__global__ __launch_bounds__(256) void attn_bwd_prep_kernel(AttnParams p, const uint16_t* __restrict__ O,
-                                                            const uint16_t* __restrict__ dO,
-                                                            const float* __restrict__ lse, int NQp, int row_blocks,
-                                                            uint16_t* __restrict__ qs, float* __restrict__ delta,
-                                                            float* __restrict__ neg, int32_t* __restrict__ tb,
-                                                            int32_t* __restrict__ rows) {
-  if ((int)blockIdx.x >= row_blocks) {
-    const int tile = ((int)blockIdx.x - row_blocks) * 4 + (threadIdx.x >> 6);
-    const int r = tile * 64 + (threadIdx.x & 63);
-    if (tile * 64 >= NQp) return;
-    const bool ok = r < p.NQ;
-    const int a1 = ok ? p.a1[r] : 0x7fffffff;
-    const int b1 = ok ? (p.b1 ? p.b1[r] : r + 1) : 0;
-    const int a2 = (ok && p.a2) ? p.T + p.a2[r] : 0x7fffffff;
-    const int b2 = (ok && p.a2) ? p.T + p.b2[r] : 0;
-    rows[r] = a1; rows[NQp + r] = b1; rows[2 * (int64_t)NQp + r] = a2; rows[3 * (int64_t)NQp + r] = b2;
-    const int v[8] = {wave_min_i(a1), wave_max_i(a1), wave_min_i(b1), wave_max_i(b1),
-                      wave_min_i(a2), wave_max_i(a2), wave_min_i(b2), wave_max_i(b2)};
-    if ((threadIdx.x & 63) == 0 && tile * 64 < p.NQ) {
+// What the dK / dV and diagonal-key kernels read next to the operands: the dQ kernel, which runs first and holds a row's q
+// and dO in registers anyway, leaves it behind.  (A prologue of its own read q, O and dO once more: 5 us and a launch at 1024
+// rows of 32 heads of 64, 26 us at 4096 of 128, 213 us at 2 x 16384 of 16 heads of 256.)
+struct BwdSide {
+  int NQp;          // rows rounded up to 128
+  uint16_t* qs;     // [Hq][NQ][D]  bf16(q * scale * log2 e)
+  float* delta;     // [Hq][NQ]     dO . O of the row
+  float* neg;       // -lse and -delta, each [Hq][NQp], zero in the padding: C operands of the dK / dV score products
+  int32_t* tb;      // [tile of 64 rows][8]  a1min, a1max, b1min, b1max, a2min, a2max, b2min, b2max
+  int32_t* rows;    // [4][NQp]     a1, b1, T + a2, T + b2 as the kernels compare them (empty: class absent, padding)
+};
+// the last two, by one wave for one tile
+__device__ __forceinline__ void interval_ends(const AttnParams& p, const BwdSide& sd, int tile, int lane) {
+  const int r = tile * 64 + lane;
+  const bool ok = r < p.NQ;
+  const int a1 = ok ? p.a1[r] : 0x7fffffff;
+  const int b1 = ok ? (p.b1 ? p.b1[r] : r + 1) : 0;
+  const int a2 = (ok && p.a2) ? p.T + p.a2[r] : 0x7fffffff;
+  const int b2 = (ok && p.a2) ? p.T + p.b2[r] : 0;
+  sd.rows[r] = a1; sd.rows[sd.NQp + r] = b1; sd.rows[2 * (int64_t)sd.NQp + r] = a2; sd.rows[3 * (int64_t)sd.NQp + r] = b2;
+  const int v[8] = {wave_min_i(a1), wave_max_i(a1), wave_min_i(b1), wave_max_i(b1),
+                    wave_min_i(a2), wave_max_i(a2), wave_min_i(b2), wave_max_i(b2)};
+  if (lane == 0 && tile * 64 < p.NQ) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) tb[tile * 8 + k] = v[k];
-    }
-    return;
-  }
-  constexpr int EPL = D / 16;
-  const int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);  // = h * NQp + i
-  const int h = (int)(item / NQp), i = (int)(item % NQp);
-  if (h >= p.Hq) return;  // (whole groups of sixteen lanes)
-  const int d0 = (threadIdx.x & 15) * EPL;
-  const bool live = i < p.NQ;
-  float acc = 0.f;
-  if (live) {
-    const int64_t row = (int64_t)i * p.Hq + h;
-    float a[EPL], b[EPL], q[EPL];
-    ld_bf16s<EPL>(O + row * D + d0, a);
-    ld_bf16s<EPL>(dO + row * D + d0, b);
-    ld_bf16s<EPL>(p.Q + (int64_t)h * p.q_hs + (int64_t)i * D + d0, q);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      acc = fmaf(a[e], b[e], acc);
-      q[e] *= p.scale_log2e;  // (the same rounded values as scale_bf16x8 gives)
-    }
-    st_bf16s<EPL>(qs + ((int64_t)h * p.NQ + i) * D + d0, q);
-  }
-  acc = row16_sum(acc);
-  if ((threadIdx.x & 15) == 0) {
-    if (live) delta[(int64_t)h * p.NQ + i] = acc;
-    neg[item] = live ? -lse[(int64_t)h * p.NQ + i] : 0.f;
-    neg[(int64_t)p.Hq * NQp + item] = live ? -acc : 0.f;
+    for (int k = 0; k < 8; ++k) sd.tb[tile * 8 + k] = v[k];
   }
 }
 
-// dQ: same tiling as the forward.
+// dQ: same tiling as the forward (a workgroup covers 128 rows: BwdSide's padding).
 //   P^T = exp2(S'^T - lse), dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
 template <int D, int NW>
 struct DqSmem {
@@ -869,8 +836,8 @@ struct DqSmem {
 
 template <int D, int NSB, int NW>
 __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_dq_kernel(
-    AttnParams p, const uint16_t* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ Delta, uint16_t* __restrict__ dQ,
-    int64_t dq_hs) {
+    AttnParams p, const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
+    BwdSide sd, uint16_t* __restrict__ dQ, int64_t dq_hs) {
   using SM = DqSmem<D, NW>;
   constexpr int TB = kBN;
   constexpr int NKK = D / 16;
@@ -899,8 +866,9 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
     i[sb] = m0 + wave * BMW + sb * 32 + col;
     ic[sb] = i[sb] < p.NQ ? i[sb] : p.NQ - 1;
     lse_i[sb] = LSE[(int64_t)h * p.NQ + ic[sb]];
-    delta_i[sb] = Delta[(int64_t)h * p.NQ + ic[sb]];
   }
+  if (h == 0)
+    for (int t = wave; t < BM / 64; t += NW) interval_ends(p, sd, m0 / 64 + t, lane);
   RowBounds<NSB> rb;
   load_bounds<NSB, NW>(p, ic, wave, lane, red, rb);
 
@@ -917,6 +885,30 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
     for (int kk = 0; kk < NKK; ++kk) {
       qf[sb][kk] = as_bf16x8(scale_bf16x8(*reinterpret_cast<const u32x4*>(qrow + kk * 16), p.scale_log2e));
       dof[sb][kk] = as_bf16x8(*reinterpret_cast<const u32x4*>(drow + kk * 16));
+    }
+    // delta, and what the kernels behind this one read
+    const uint16_t* orow = O + ((int64_t)ic[sb] * p.Hq + h) * D + g * 8;
+    float dot = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+      float o8[8], d8[8];
+      unpack8(*reinterpret_cast<const u32x4*>(orow + kk * 16), o8);
+      unpack8(__builtin_bit_cast(u32x4, dof[sb][kk]), d8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot = fmaf(o8[e], d8[e], dot);
+    }
+    delta_i[sb] = half_swap_sum(dot);
+    const bool live = i[sb] < p.NQ;
+    if (live) {
+      uint16_t* qrow_s = sd.qs + ((int64_t)h * p.NQ + i[sb]) * D + g * 8;
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk)
+        *reinterpret_cast<u32x4*>(qrow_s + kk * 16) = __builtin_bit_cast(u32x4, qf[sb][kk]);
+    }
+    if (g == 0) {
+      if (live) sd.delta[(int64_t)h * p.NQ + i[sb]] = delta_i[sb];
+      sd.neg[(int64_t)h * sd.NQp + i[sb]] = live ? -lse_i[sb] : 0.f;
+      sd.neg[((int64_t)p.Hq + h) * sd.NQp + i[sb]] = live ? -delta_i[sb] : 0.f;
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) { nlse[sb][r] = -lse_i[sb]; ndel[sb][r] = -delta_i[sb]; }
@@ -1131,35 +1123,46 @@ namespace spx {
 
 // dK[kvh, c, :] = scaling * sum of the partial results of the head units of kvh (n_hu / Hkv of them in each of n_sum
 // sets), dV likewise (no scaling); bf16 out.  `accumulate`: what dK / dV hold is added (in fp32, one rounding).
-__global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(
-    const float* __restrict__ dKp, const float* __restrict__ dVp, int NKV, int D, int n_hu, int n_sum, int Hkv,
-    float scaling, uint16_t* __restrict__ dK, int64_t dk_hs, uint16_t* __restrict__ dV, int64_t dv_hs,
-    int accumulate) {
-  const int64_t per_head = (int64_t)NKV * D / 4;  // float4 items
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= per_head * Hkv) return;
+struct DkvSum {
+  const float *dKp, *dVp;
+  int NKV, n_hu, n_sum, Hkv;
+  float scaling;
+  uint16_t* dK; int64_t dk_hs;
+  uint16_t* dV; int64_t dv_hs;
+  int accumulate;
+};
+template <int D>
+__device__ __forceinline__ void dkv_sum(const DkvSum& a, int64_t idx) {
+  const int64_t per_head = (int64_t)a.NKV * D / 4;  // float4 items
+  if (idx >= per_head * a.Hkv) return;
   const int kvh = (int)(idx / per_head);
   const int64_t off = (idx % per_head) * 4;
-  const int units = n_hu / Hkv;
+  const int units = a.n_hu / a.Hkv;
   f32x4 sk = {0, 0, 0, 0}, sv = {0, 0, 0, 0};
-  for (int s = 0; s < n_sum; ++s)
+  for (int s = 0; s < a.n_sum; ++s)
     for (int u = 0; u < units; ++u) {
-      const int64_t base = ((int64_t)(s * n_hu + kvh * units + u) * NKV) * D + off;
-      sk += *reinterpret_cast<const f32x4*>(dKp + base);
-      sv += *reinterpret_cast<const f32x4*>(dVp + base);
+      const int64_t base = ((int64_t)(s * a.n_hu + kvh * units + u) * a.NKV) * D + off;
+      sk += *reinterpret_cast<const f32x4*>(a.dKp + base);
+      sv += *reinterpret_cast<const f32x4*>(a.dVp + base);
     }
-  sk *= scaling;
+  sk *= a.scaling;
   u32x2 wk, wv;
-  if (accumulate) {
-    wk = *reinterpret_cast<const u32x2*>(dK + (int64_t)kvh * dk_hs + off);
-    wv = *reinterpret_cast<const u32x2*>(dV + (int64_t)kvh * dv_hs + off);
+  u32x2* const kp = reinterpret_cast<u32x2*>(a.dK + (int64_t)kvh * a.dk_hs + off);
+  u32x2* const vp = reinterpret_cast<u32x2*>(a.dV + (int64_t)kvh * a.dv_hs + off);
+  if (a.accumulate) {
+    wk = *kp;
+    wv = *vp;
     sk.x += bf16_lo(wk.x); sk.y += bf16_hi(wk.x); sk.z += bf16_lo(wk.y); sk.w += bf16_hi(wk.y);
     sv.x += bf16_lo(wv.x); sv.y += bf16_hi(wv.x); sv.z += bf16_lo(wv.y); sv.w += bf16_hi(wv.y);
   }
   wk.x = pack_bf16x2(sk.x, sk.y); wk.y = pack_bf16x2(sk.z, sk.w);
   wv.x = pack_bf16x2(sv.x, sv.y); wv.y = pack_bf16x2(sv.z, sv.w);
-  *reinterpret_cast<u32x2*>(dK + (int64_t)kvh * dk_hs + off) = wk;
-  *reinterpret_cast<u32x2*>(dV + (int64_t)kvh * dv_hs + off) = wv;
+  *kp = wk;
+  *vp = wv;
+}
+template <int D>
+__global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(DkvSum a) {
+  dkv_sum<D>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 // dK / dV of the TTT diagonal keys (j, i), j >= 1: sixteen lanes per (position, K/V head)
@@ -1170,19 +1173,25 @@ __global__ __launch_bounds__(256) void attn_dkv_reduce_kernel(
 // MAXG = query heads per K/V head whose rows are kept in registers: a group of at most MAXG heads
 // reads its query / output-gradient rows once for all diagonals; a wider group walks its heads in
 // passes of MAXG inside every diagonal (rows re-read per diagonal, from L2).
+// The first sum_blocks workgroups add up the partial results of the other keys (dkv_sum): both are short (5 us each at
+// 1024 rows of the 1B shape, 14 + 18 at 3001 of the 8B shape) and share no result, so one launch takes as long as the longer.
 template <int D, int MAXG>
 __global__ __launch_bounds__(256) void ttt_attn_bwd_diag_kernel(
     const uint16_t* __restrict__ Q, int64_t q_hs, const uint16_t* __restrict__ K, int64_t k_hs,
     const uint16_t* __restrict__ V, int64_t v_hs, const uint16_t* __restrict__ dO,
     const float* __restrict__ LSE, const float* __restrict__ Delta, int T, int n_extra, int Hq,
     int Hkv, float scale_log2e, float scaling, uint16_t* dK, int64_t dk_hs, uint16_t* dV,
-    int64_t dv_hs, int accumulate) {
+    int64_t dv_hs, int accumulate, DkvSum sum, int sum_blocks) {
+  if ((int)blockIdx.x < sum_blocks) {
+    dkv_sum<D>(sum, (int64_t)blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
   constexpr int EPL = D / 16;
   // item = kvh * T + i: neighbouring 16-lane rows take neighbouring positions of one K/V head, so
   // their key / value / gradient rows are contiguous in memory.  The tail clamps (no early
   // return: the DPP sums need whole rows of lanes)
   const int64_t n_items = (int64_t)T * Hkv;
-  const int64_t raw = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + ((threadIdx.x & 63) >> 4);
+  const int64_t raw = (((int64_t)blockIdx.x - sum_blocks) * 4 + (threadIdx.x >> 6)) * 4 + ((threadIdx.x & 63) >> 4);
   const bool live = raw < n_items;
   const int64_t item = live ? raw : n_items - 1;
   const int kvh = (int)(item / T), i = (int)(item % T);
@@ -1389,11 +1398,15 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
   AttnParams ps = p;
   ps.Q = qs;
   ps.q_hs = (int64_t)p.NQ * D;
-  const int row_blocks = (int)(((int64_t)p.Hq * NQp + 15) / 16);
-  hipLaunchKernelGGL(attn_bwd_prep_kernel<D>, dim3((unsigned)(row_blocks + (NQp / 64 + 3) / 4)), dim3(256), 0, st, p, Op,
-                     dOp, lse, NQp, row_blocks, qs, delta, neg, tb, mrows);
+  // (byte offsets of dO's rows are 32 bits, without a sign; the rows that fill the last tile count)
+  if (D > 128 ? (int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31) : ((int64_t)p.NQ + 64) * p.Hq * D * 2 >= (1ll << 32)) {
+    last_error() = std::string(fn) + ": queries must span less than " + (D > 128 ? "2" : "4") + " GiB";
+    return SPX_ERR_ARG;
+  }
+  const BwdSide side = {NQp, qs, delta, neg, tb, mrows};
 
   constexpr int BM = 32 * kDqNSB * kDqNW;
+  static_assert(BM == 128, "the rows of BwdSide are rounded up to a workgroup's");
   const int n_qb = (p.NQ + BM - 1) / BM;
   {
     constexpr int dq_smem = DqSmem<D, kDqNW>::kBytes;
@@ -1406,34 +1419,30 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
                                     dq_lds_set, fn))
       return rc;
     hipLaunchKernelGGL((attn_bwd_dq_kernel<D, kDqNSB, kDqNW>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kDqNW), dq_smem,
-                       st, p, dOp, lse, delta, dQp, dq_hs);
+                       st, p, Op, dOp, lse, side, dQp, dq_hs);
   }
 
-  // (byte offsets of dO's rows are 32 bits, without a sign; the rows that fill the last tile count)
-  if (D > 128 ? (int64_t)p.NQ * p.Hq * D * 2 >= (1ll << 31) : ((int64_t)p.NQ + 64) * p.Hq * D * 2 >= (1ll << 32)) {
-    last_error() = std::string(fn) + ": queries must span less than " + (D > 128 ? "2" : "4") + " GiB";
-    return SPX_ERR_ARG;
-  }
   static std::atomic<uint64_t> dkv_lds_set;  // per head_dim instantiation, one bit per device
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<D>), DkvCfg<D>::kBytes,
                                   dkv_lds_set, fn))
     return rc;
   hipLaunchKernelGGL((attn_bwd_dkv_kernel<D>), dim3((unsigned)(pl.n_k * pl.n_hu)), dim3(512), DkvCfg<D>::kBytes, st,
                      ps, dOp, NQp, neg, mrows, tb, pl, dkp, dvp);
-  const int64_t items = (int64_t)p.NKV * D / 4 * p.Hkv;
-  hipLaunchKernelGGL(attn_dkv_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, dkp,
-                     dvp, p.NKV, D, pl.n_hu, pl.windows, p.Hkv, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate);
-  if (p.n_extra > 0) {
-    const dim3 dgrid((unsigned)(((int64_t)p.T * p.Hkv + 15) / 16));
+  const int sum_blocks = (int)(((int64_t)p.NKV * D / 4 * p.Hkv + 255) / 256);
+  const DkvSum sum = {dkp, dvp, p.NKV, pl.n_hu, pl.windows, p.Hkv, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate};
+  if (p.n_extra == 0) {
+    hipLaunchKernelGGL(attn_dkv_reduce_kernel<D>, dim3((unsigned)sum_blocks), dim3(256), 0, st, sum);
+  } else {
+    const dim3 dgrid((unsigned)(sum_blocks + ((int64_t)p.T * p.Hkv + 15) / 16));
     // eight heads per K/V head in registers where they fit (head_dim <= 128), else four
     if (D <= 128 && p.Hq / p.Hkv > 4)
       hipLaunchKernelGGL((ttt_attn_bwd_diag_kernel<D, (D <= 128 ? 8 : 4)>), dgrid, dim3(256), 0, st, ps.Q,
                          ps.q_hs, p.K, p.k_hs, p.V, p.v_hs, dOp, lse, delta, p.T, p.n_extra, p.Hq, p.Hkv,
-                         1.f, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate);
+                         1.f, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate, sum, sum_blocks);
     else
       hipLaunchKernelGGL((ttt_attn_bwd_diag_kernel<D, 4>), dgrid, dim3(256), 0, st, ps.Q, ps.q_hs, p.K,
                          p.k_hs, p.V, p.v_hs, dOp, lse, delta, p.T, p.n_extra, p.Hq, p.Hkv,
-                         1.f, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate);
+                         1.f, kLn2, dKp, dk_hs, dVp, dv_hs, accumulate, sum, sum_blocks);
   }
   return check_launch(fn);
 }
