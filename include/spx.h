@@ -322,6 +322,27 @@ int spx_block_reduce(const float* loss, const int32_t* argmax_draft,
                      int32_t block_size, float* out, float* correct,
                      float* total, float* row_weight, void* stream);
 
+/* spx_block_reduce with the term's place in the loss and the step's metrics in the same launch.  pos_weight NULL: the
+ * weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0, or exp(-s / gamma) where blocks start at their anchor
+ * (from_anchor; losses/utils.py:17-48).  out [9 + 2 * block_size]: the two scalars of spx_block_reduce, then
+ *   out[2] = *total_out = factor * out[0] (+ *total_in),  out[3], out[4] = matches, rows over the slots that count (all,
+ *   or all but slot 0),  out[5] = sum of the running products of their accuracies,  out[6 .. 8] = 1,
+ *   out[9 + s], out[9 + block_size + s] = matches, rows of slot s. */
+int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target, const void* mask,
+                    int mask_kind, const float* pos_weight, float gamma, int from_anchor, int64_t rows,
+                    int32_t block_size, float factor, const float* total_in, float* total_out, float* out,
+                    float* row_weight, void* stream);
+
+/* The inputs of an anchored-block step (models/dflash/core.py:264-271,330-439) in one launch, n_q = n_anchors *
+ * block_size rows: ids[r] = the anchor's token in slot 0, mask_token in the others; kv_pos [T + n_q] = positions, then
+ * positions[anchor] + slot; target_row[r] = the row whose target row r predicts (its own, or the one before it);
+ * aligned[r] = loss_mask of its own row, 0 for invalid anchors and (unless from_anchor) in slot 0, NaN for a valid anchor
+ * whose block leaves the sequence.  Anchors below 0 count from the end. */
+int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size, int64_t T,
+                      int64_t mask_token, const int64_t* input_ids, const int64_t* positions, const void* loss_mask,
+                      int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos, int64_t* target_row,
+                      float* aligned, void* stream);
+
 /* ---------------------------------------------------------------- TTT attention
  * row_lo[i] = lowest context key visible to query i: the interval form
  * row_lo[i] <= c <= i of the step-0 part of create_combined_mask_mod

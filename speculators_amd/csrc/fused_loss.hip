@@ -1289,19 +1289,35 @@ __global__ __launch_bounds__(kLossThreads) void row_tokens_kernel(const int32_t*
   }
 }
 
+// What spx_block_total adds to the reduction of a block batch (scalars == nullptr: nothing).
+struct BlockTotal {
+  float gamma;            // > 0: the weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0; from_anchor: exp(-s / gamma)
+  int from_anchor;
+  float factor;           // the term's weight in the loss
+  const float* total_in;  // loss so far (nullptr: none)
+  float* total_out;
+  float* scalars;
+};
+
 __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
     const float* __restrict__ loss, const int32_t* __restrict__ pred,
     const int32_t* __restrict__ tgt, const void* __restrict__ mask, int mask_kind,
     const float* __restrict__ pos_weight, int64_t rows, int block_size, float* __restrict__ out,
-    float* __restrict__ correct, float* __restrict__ total, float* __restrict__ row_weight) {
+    float* __restrict__ correct, float* __restrict__ total, float* __restrict__ row_weight, BlockTotal bt) {
   __shared__ float fl[kReduceThreads / 64];
-  extern __shared__ int slots[];  // [2 * block_size]
+  extern __shared__ int slots[];  // [2 * block_size], and a weight per slot behind them
+  float* const decay = reinterpret_cast<float*>(slots + 2 * block_size);
+  const bool by_slot = bt.gamma > 0.f;
   for (int i = threadIdx.x; i < 2 * block_size; i += kReduceThreads) slots[i] = 0;
+  if (by_slot)
+    for (int i = threadIdx.x; i < block_size; i += kReduceThreads)
+      decay[i] = bt.from_anchor ? expf(-(float)i / bt.gamma) : i == 0 ? 0.f : expf(-(float)(i - 1) / bt.gamma);
   __syncthreads();
+  auto weight = [&](int64_t r) { return by_slot ? decay[r % block_size] : pos_weight ? pos_weight[r] : 1.f; };
   float lsum = 0.f, msum = 0.f;
   for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
     float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
-    float w = pos_weight ? pos_weight[r] : 1.f;
+    float w = weight(r);
     if (m != 0.f) {
       int s = (int)(r % block_size);
       atomicAdd(&slots[block_size + s], 1);
@@ -1319,13 +1335,58 @@ __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
     correct[i] = (float)slots[i];
     total[i] = (float)slots[block_size + i];
   }
+  if (bt.scalars && threadIdx.x == 0) {
+    const float part = bt.factor * (lsum * inv), sum = bt.total_in ? *bt.total_in + part : part;
+    *bt.total_out = sum;
+    // the step's metrics: what a dozen one-element kernels did
+    float hits = 0.f, rows_in = 0.f, run = 1.f, eal = 0.f;
+    for (int i = bt.from_anchor ? 0 : 1; i < block_size; ++i) {
+      const float c = (float)slots[i], t = (float)slots[block_size + i];
+      hits += c;
+      rows_in += t;
+      run *= c / fmaxf(t, 1.f);
+      eal += run;
+    }
+    bt.scalars[0] = sum;
+    bt.scalars[1] = hits;
+    bt.scalars[2] = rows_in;
+    bt.scalars[3] = eal;
+    bt.scalars[4] = bt.scalars[5] = bt.scalars[6] = 1.f;
+  }
   if (row_weight) {
     for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
       float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
-      float w = pos_weight ? pos_weight[r] : 1.f;
+      float w = weight(r);
       row_weight[r] = m * w * inv;
     }
   }
+}
+
+// One thread per row of the draft: the inputs of an anchored-block step (models/dflash/core.py:264-271,330-439)
+__global__ __launch_bounds__(256) void dflash_inputs_kernel(
+    const int64_t* __restrict__ anchors, const uint8_t* __restrict__ valid, int n_q, int block_size, int64_t T,
+    int64_t mask_token, const int64_t* __restrict__ input_ids, const int64_t* __restrict__ positions,
+    const void* __restrict__ loss_mask, int mask_kind, int from_anchor, int64_t* __restrict__ ids,
+    int64_t* __restrict__ kv_pos, int64_t* __restrict__ target_row, float* __restrict__ aligned) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < T) {
+    kv_pos[i] = positions[i];
+    return;
+  }
+  const int64_t r = i - T;
+  if (r >= n_q) return;
+  const int j = (int)(r / block_size), s = (int)(r % block_size);
+  int64_t a = anchors[j];
+  if (a < 0) a += T;
+  const bool inside = a >= 0 && a + s < T;
+  a = min(max(a, (int64_t)0), T - 1);
+  const int64_t row = min(a + s, T - 1);
+  ids[r] = s == 0 ? input_ids[a] : mask_token;
+  kv_pos[i] = positions[a] + s;
+  target_row[r] = from_anchor ? row : row > 0 ? row - 1 : T - 1;
+  // (a block that leaves the sequence shows in the loss)
+  const float m = mask_value(loss_mask, mask_kind, row) * (valid[j] ? 1.f : 0.f);
+  aligned[r] = !inside && valid[j] ? __uint_as_float(0x7fc00000u) : (!from_anchor && s == 0) ? 0.f : m;
 }
 
 // ---- dispatch ----------------------------------------------------------------
@@ -1747,18 +1808,54 @@ extern "C" int spx_row_tokens(const int32_t* known, int64_t n, const void* rows,
   return check_launch(__func__);
 }
 
+static int block_reduce(const char* fname, const float* loss, const int32_t* argmax_draft,
+                        const int32_t* argmax_target, const void* mask, int mask_kind, const float* pos_weight,
+                        int64_t rows, int32_t block_size, float* out, float* correct, float* total, float* row_weight,
+                        const BlockTotal& bt, void* stream) {
+#define SPX_REQ_FN(cond, what) do { if (!(cond)) return spx::fail_arg(fname, what); } while (0)
+  SPX_REQ_FN(rows >= 0 && rows < (1ll << 24), "0 <= rows < 2^24");
+  SPX_REQ_FN(block_size > 0 && block_size <= 4096, "0 < block_size <= 4096");
+  SPX_REQ_FN(loss && argmax_draft && argmax_target && out && correct && total, "null buffer");
+  SPX_REQ_FN(!mask || kind_ok(mask_kind), "unknown mask element kind");
+#undef SPX_REQ_FN
+  hipLaunchKernelGGL(block_reduce_kernel, dim3(1), dim3(kReduceThreads),
+                     (2 * sizeof(int) + sizeof(float)) * block_size, reinterpret_cast<hipStream_t>(stream), loss,
+                     argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
+                     correct, total, row_weight, bt);
+  return check_launch(fname);
+}
+
 extern "C" int spx_block_reduce(const float* loss, const int32_t* argmax_draft,
                                 const int32_t* argmax_target, const void* mask, int mask_kind,
                                 const float* pos_weight, int64_t rows, int32_t block_size,
                                 float* out, float* correct, float* total, float* row_weight,
                                 void* stream) {
-  SPX_REQUIRE(rows >= 0 && rows < (1ll << 24), "0 <= rows < 2^24");
-  SPX_REQUIRE(block_size > 0 && block_size <= 4096, "0 < block_size <= 4096");
-  SPX_REQUIRE(loss && argmax_draft && argmax_target && out && correct && total, "null buffer");
-  SPX_REQUIRE(!mask || kind_ok(mask_kind), "unknown mask element kind");
-  hipLaunchKernelGGL(block_reduce_kernel, dim3(1), dim3(kReduceThreads),
-                     2 * block_size * sizeof(int), reinterpret_cast<hipStream_t>(stream), loss,
-                     argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
-                     correct, total, row_weight);
+  return block_reduce(__func__, loss, argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
+                      correct, total, row_weight, BlockTotal{}, stream);
+}
+
+extern "C" int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target,
+                               const void* mask, int mask_kind, const float* pos_weight, float gamma, int from_anchor,
+                               int64_t rows, int32_t block_size, float factor, const float* total_in,
+                               float* total_out, float* out, float* row_weight, void* stream) {
+  SPX_REQUIRE(total_out && out && row_weight, "null buffer");
+  SPX_REQUIRE(pos_weight || gamma > 0.f, "a weight per row or a positive gamma");
+  const BlockTotal bt = {pos_weight ? 0.f : gamma, from_anchor, factor, total_in, total_out, out + 2};
+  return block_reduce(__func__, loss, argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
+                      out + 9, out + 9 + block_size, row_weight, bt, stream);
+}
+
+extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
+                                 int64_t T, int64_t mask_token, const int64_t* input_ids, const int64_t* positions,
+                                 const void* loss_mask, int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos,
+                                 int64_t* target_row, float* aligned, void* stream) {
+  SPX_REQUIRE(T > 0 && T < (1ll << 30) && n_anchors >= 0 && block_size > 0 && n_anchors * block_size < (1ll << 30),
+              "sizes out of range");
+  SPX_REQUIRE(input_ids && positions && loss_mask && kv_pos && kind_ok(mask_kind), "null buffer or unknown mask kind");
+  SPX_REQUIRE(n_anchors == 0 || (anchors && valid && ids && target_row && aligned), "null buffer");
+  const int64_t n_q = n_anchors * block_size;
+  hipLaunchKernelGGL(dflash_inputs_kernel, dim3((unsigned)((T + n_q + 255) / 256)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), anchors, valid, (int)n_q, block_size, T, mask_token,
+                     input_ids, positions, loss_mask, mask_kind, from_anchor, ids, kv_pos, target_row, aligned);
   return check_launch(__func__);
 }

@@ -21,6 +21,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _lib
 from . import attention as A
 from . import fused_ops as FO
 from . import gemm
@@ -222,6 +223,31 @@ class DFlashDraftModel(nn.Module):
         """``x @ weight.T`` on the MFMA kernel of this library (fc, lm_head, verifier head)."""
         return gemm.linear_staged(x, self._stager.get(weight), hip=True)
 
+    def _inputs(self, input_ids, position_ids, loss_mask, anchors, valid, t: int):
+        """``(ids [1, n_q], q_pos [n_q], kv_pos [t + n_q], target rows [n_q], aligned loss mask [1, n_q])`` of the blocks
+        that start at ``anchors`` (models/dflash/core.py:264-271,330-439)."""
+        dev, bs, cfg = input_ids.device, self.block_size, self.config
+        n_q = anchors.numel() * bs
+
+        def row(x, dtype=torch.int64):
+            x = x.reshape(-1) if dtype is None else x.reshape(-1).to(dtype)
+            return x if x.is_contiguous() else x.contiguous()
+
+        ids, pos, mask = row(input_ids), row(position_ids), row(loss_mask, None)
+        if not ids.numel() == pos.numel() == mask.numel() == t or valid.numel() != anchors.numel():
+            raise ValueError(f"input_ids, position_ids and loss_mask must hold {t} entries, the anchors one flag each")
+        if mask.dtype not in _lib.KIND_CODE:
+            mask = mask.float()
+        ints = torch.empty(t + 3 * n_q, device=dev, dtype=torch.int64)
+        kv_pos, out_ids, idx = ints[:t + n_q], ints[t + n_q:t + 2 * n_q], ints[t + 2 * n_q:]
+        aligned = torch.empty(1, n_q, device=dev, dtype=torch.float32)
+        _lib.call("spx_dflash_inputs", row(anchors.to(dev)), row(valid.to(dev), torch.bool), anchors.numel(), bs, t,
+                  int(self.mask_token_id), ids, pos, mask, _lib.kind_code(mask), int(cfg.sample_from_anchor), out_ids,
+                  kv_pos, idx, aligned, _lib.stream_ptr(dev))
+        if valid.dtype != torch.bool:  # (weights instead of flags)
+            aligned *= valid.to(dev, torch.float32).reshape(-1).repeat_interleave(bs)
+        return out_ids.view(1, n_q), kv_pos[t:], kv_pos, idx, aligned
+
     def forward(self, hidden_states, input_ids, loss_mask, verifier_last_hidden_states,
                 document_ids, position_ids=None, loss_config: L.LossConfig | None = None,
                 gamma: float = 4.0, max_anchors: int = 512,
@@ -246,19 +272,12 @@ class DFlashDraftModel(nn.Module):
         sw_mask = (A.create_dflash_mask(doc, t, anchor_pos, bs, cfg.sliding_window,
                                         cfg.sliding_window_non_causal)
                    if self.uses_sliding_window_attn else None)
-        n_q = anchor_pos.numel() * bs
-        ids = torch.full((1, n_q), self.mask_token_id, dtype=torch.long, device=device)
-        ids[:, ::bs] = input_ids[:, anchor_pos]
+        ids, q_pos, kv_pos, idx, aligned = self._inputs(input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t)
         with torch.no_grad():
             noise = F.embedding(ids, self.embed_tokens.weight).to(hidden_states.dtype)
         ctx = self.hidden_norm(self._linear(hidden_states, self.fc.weight))
-        block_pos = get_base_indices_for_anchored_blocks(position_ids[0, anchor_pos], bs)
-        kv_pos = torch.cat([position_ids.reshape(-1), block_pos]).to(torch.int64).contiguous()
-        q_pos = block_pos.to(torch.int64).contiguous()
         inv_freq = self._rotary.select(device, self._rotary.top(kv_pos))
-        block_idx = get_base_indices_for_anchored_blocks(anchor_pos, bs)
         with torch.no_grad():
-            idx = block_idx if cfg.sample_from_anchor else (block_idx - 1) % t
             targets = self._linear(self.verifier_norm(verifier_last_hidden_states[:, idx]),
                                    self.verifier_lm_head.weight)
         normed = None
@@ -275,10 +294,6 @@ class DFlashDraftModel(nn.Module):
             logits = MT.Head(normed, head.w, head.wt)
         else:
             logits = gemm.linear_staged(normed, head, hip=True)
-        aligned = loss_mask.clone()[:, block_idx]
-        aligned = aligned * anchor_valid.repeat_interleave(bs).unsqueeze(0).to(aligned.dtype)
-        if not cfg.sample_from_anchor:
-            aligned[:, ::bs] = 0
         loss, metrics = MT.dflash_compute_metrics(
             logits, targets, aligned, bs, gamma=gamma, loss_config=loss_config,
             per_position_loss_weight=per_position_loss_weight, dpace_alpha=dpace_alpha,

@@ -265,7 +265,8 @@ def normed_forward(s: NormedLayer, x, n, context, gain_in, gain_q, gain_k, gain_
     rstd_in = None
     if context is not None:
         c2 = _flat(context)
-        both = torch.cat((c2, _flat(n)))
+        n2 = _flat(n)
+        both = _lib.native().cat_bf16(c2, n2) if c2.is_contiguous() and n2.is_contiguous() else torch.cat((c2, n2))
         n2 = both[c2.shape[0]:]
         q_tok, kv_tok = gemm._project(n2, s.wq), gemm._project(both, s.wkv)
     else:

@@ -335,6 +335,34 @@ class MeanTerm:
         return total, row_weight
 
 
+@dataclass
+class BlockTerm:
+    """``MeanTerm`` for a batch of anchored blocks (``spx_block_total``): the weighted masked mean of one term, its
+    ``factor`` in the loss, and ``out`` (f32 ``[9 + 2 * block_size]``), which receives the step's scalars.  ``row_weights``:
+    weights from the masked row losses (D-PACE) in the place of the exponential decay over the slots."""
+
+    mask: torch.Tensor
+    block_size: int
+    gamma: float
+    from_anchor: bool
+    factor: float
+    out: torch.Tensor
+    row_weights: Callable | None = None
+
+    def reduce(self, loss, am_d, am_t, counts, total_in):
+        """As ``MeanTerm.reduce`` (``counts``: none, blocks have no acceptance chain)."""
+        n, dev = loss.numel(), loss.device
+        pos = None
+        if self.row_weights is not None:
+            pos = self.row_weights(loss.detach() * self.mask.to(torch.float32)).contiguous()
+        row_weight = torch.empty(n, device=dev, dtype=torch.float32)
+        total = torch.empty((), device=dev, dtype=torch.float32)
+        _lib.call("spx_block_total", loss, am_d, am_t, self.mask, _lib.kind_code(self.mask), pos, float(self.gamma),
+                  int(self.from_anchor), n, self.block_size, self.factor, total_in, total, self.out, row_weight,
+                  _lib.stream_ptr(dev))
+        return total, row_weight
+
+
 def _unit_rows_backward(saved, g32, factor: float, total_rows: int):
     """dx of the frozen head from the unit-weight logits gradient of the live rows that the row pass left behind."""
     from .gemm import matmul_nt
@@ -362,15 +390,22 @@ class _HeadStepLoss(torch.autograd.Function):
         logits = matmul_nt(x2, weight)
         ctx.op, ctx.total_rows, ctx.factor = op, logits.shape[0], mean.factor
         xs = logits[:n_rows]
-        ctx.one_pass = (known is not None or targets is not None) and _one_pass_ok(op, xs, targets, step)
+        blocks = isinstance(mean, BlockTerm)
+        ctx.one_pass = ((known is not None or targets is not None) and _one_pass_ok(op, xs, targets, step)
+                        and (not blocks or xs.shape[1] >= TERMS_MIN_VOCAB))
         if ctx.one_pass:
-            total, _, am_d, am_t, lse_t, packed, row_map, count, row_weight = _loss_step(op, xs, targets, known, step, mean,
-                                                                                      total_in)
+            total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight = _loss_step(
+                op, xs, targets, known, step, None if blocks else mean, total_in)
+            if blocks:
+                total, row_weight = mean.reduce(loss, am_d, am_t, None, total_in)
             ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
         else:
-            step.counts = torch.zeros(3, device=x2.device, dtype=torch.int32)
+            if blocks:
+                step = None
+            else:
+                step.counts = torch.zeros(3, device=x2.device, dtype=torch.int32)
             loss, lse_d, lse_t, extra, am_d, am_t, x, y = fused_loss_forward(op, xs, targets, known, step)
-            total, row_weight = mean.reduce(loss, am_d, am_t, step.counts, total_in)
+            total, row_weight = mean.reduce(loss, am_d, am_t, None if blocks else step.counts, total_in)
             ctx.save_for_backward(x, None if op == OP_CE else y, lse_d, lse_t, extra, am_t, weight_t, row_weight)
         ctx.mark_non_differentiable(am_d, am_t, lse_t, logits)
         ctx.set_materialize_grads(False)

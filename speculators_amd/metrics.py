@@ -340,25 +340,20 @@ def argmax_rows(logits: torch.Tensor) -> torch.Tensor:
 
 
 class _BlockReduce(torch.autograd.Function):
+    """(row_loss [n] f32, total_in) -> total_in + the term (``losses.BlockTerm``); d / d row_loss = factor * row_weight."""
+
     @staticmethod
-    def forward(ctx, row_loss, am_d, am_t, mask, pos_weight, block_size, out, correct, total):
-        n = row_loss.numel()
-        row_loss = row_loss.reshape(-1).contiguous()
-        row_weight = torch.empty(n, device=row_loss.device, dtype=torch.float32)
-        _lib.call(
-            "spx_block_reduce", row_loss, am_d, am_t, mask,
-            _lib.kind_code(mask), pos_weight, n, int(block_size), out,
-            correct, total, row_weight,
-            _lib.stream_ptr(row_loss.device),
-        )
+    def forward(ctx, row_loss, total_in, am_d, am_t, term):
+        total, row_weight = term.reduce(row_loss.reshape(-1).contiguous(), am_d, am_t, None, total_in)
         ctx.save_for_backward(row_weight)
-        ctx.shape = row_loss.shape
-        return out[0].clone()
+        ctx.shape, ctx.factor = row_loss.shape, term.factor
+        return total
 
     @staticmethod
     def backward(ctx, g):
         (row_weight,) = ctx.saved_tensors
-        return (row_weight * g).view(ctx.shape), None, None, None, None, None, None, None, None
+        scaled = g if ctx.factor == 1.0 else g * ctx.factor
+        return (row_weight * scaled).view(ctx.shape), g if ctx.needs_input_grad[1] else None, None, None, None
 
 
 def dflash_loss_decay(pos_idx: torch.Tensor, gamma: float, sample_from_anchor: bool = False):
@@ -404,51 +399,41 @@ def dflash_compute_metrics(logits, targets, loss_mask, block_size: int = 1, gamm
         else:
             logits = logits.materialize()
     dev = logits.device
-    n = logits.shape[1]
     mask1 = _as_mask(loss_mask)
-    pos = torch.arange(n, device=dev) % block_size
-    total_loss = None
+    total = first = None
     terms = {}
-    multi = len(loss_config) > 1
-    correct = total = None
     for ti, (name, (fn, w)) in enumerate(loss_config.items()):
         op = L.PRIMITIVE_OP.get(name)
+        out = torch.empty(9 + 2 * block_size, device=dev, dtype=torch.float32)
+        dpace = (lambda rows: dpace_loss_decay(rows, mask1, block_size, dpace_alpha)
+                 ) if per_position_loss_weight == "dpace" else None
+        term = L.BlockTerm(mask1, block_size, gamma, sample_from_anchor, float(w), out, dpace)
         if head is not None:
-            rows, am_d, am_t, _, head.logits = L.head_fused_rows(
-                op, head.x, head.weight, head.weight_t, targets)
-        elif fn is L._HIP_LOSS_FN_MAP.get(name) and op is not None:
-            rows, am_d, am_t, _ = L.fused_rows(op, logits, targets)
+            total, _, _, _, head.logits = L.head_step_loss(
+                op, head.x, head.weight, head.weight_t, targets, None, head.x.shape[1],
+                L.StepPass(mask=mask1, grad_in_pass=True), term, total)
         else:
-            rows = fn(logits, targets)
-            _, am_d, am_t, _ = L.fused_rows(L.OP_CE, logits.detach(), targets)
-        if per_position_loss_weight == "dpace":
-            masked = rows.detach().reshape(-1) * mask1.to(torch.float32)
-            pw = dpace_loss_decay(masked, mask1, block_size, dpace_alpha)
-        else:
-            pw = dflash_loss_decay(pos, gamma, sample_from_anchor)
-        out = torch.empty(2, device=dev, dtype=torch.float32)
-        c = torch.empty(block_size, device=dev, dtype=torch.float32)
-        t = torch.empty(block_size, device=dev, dtype=torch.float32)
-        term = _BlockReduce.apply(rows.reshape(-1), am_d.reshape(-1), am_t.reshape(-1), mask1,
-                                  pw.contiguous(), block_size, out, c, t)
+            if fn is L._HIP_LOSS_FN_MAP.get(name) and op is not None:
+                rows, am_d, am_t, _ = L.fused_rows(op, logits, targets)
+            else:
+                rows = fn(logits, targets)
+                _, am_d, am_t, _ = L.fused_rows(L.OP_CE, logits.detach(), targets)
+            total = _BlockReduce.apply(rows.reshape(-1), total, am_d.reshape(-1), am_t.reshape(-1), term)
         if ti == 0:
-            correct, total = c, t
-        if multi:
-            terms[f"{name}_loss"] = term.detach()
-        total_loss = w * term if total_loss is None else total_loss + w * term
+            first = out
+        if len(loss_config) > 1:
+            terms[f"{name}_loss"] = out[0], out[6]
 
-    one = torch.ones((), device=dev)
-    m = {"loss_sum": total_loss.detach().clone(), "loss_total": one}
-    for tname, tval in terms.items():
+    one = first[7]
+    m = {"loss_sum": out[2], "loss_total": one}
+    for tname, (tval, tone) in terms.items():
         m[f"{tname}_sum"] = tval
-        m[f"{tname}_total"] = one.clone()
-    first = 0 if sample_from_anchor else 1
-    m["full_acc_sum"] = correct[first:].sum()
-    m["full_acc_total"] = total[first:].sum()
-    acc = correct[first:] / total[first:].clamp(min=1.0)
-    m["eal_sum"] = torch.cumprod(acc, dim=0).sum() if acc.numel() else torch.zeros((), device=dev)
-    m["eal_total"] = one.clone()
-    for s in range(first, block_size):
-        m[f"position_{s}_acc_sum"] = correct[s]
-        m[f"position_{s}_acc_total"] = total[s]
-    return total_loss, m
+        m[f"{tname}_total"] = tone
+    m["full_acc_sum"] = first[3]
+    m["full_acc_total"] = first[4]
+    m["eal_sum"] = first[5]
+    m["eal_total"] = first[8]
+    for s in range(0 if sample_from_anchor else 1, block_size):
+        m[f"position_{s}_acc_sum"] = first[9 + s]
+        m[f"position_{s}_acc_total"] = first[9 + block_size + s]
+    return total, m
