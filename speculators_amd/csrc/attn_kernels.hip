@@ -130,8 +130,9 @@ __device__ __forceinline__ u32x4 scale_bf16x8(u32x4 raw, float c) {
 }
 
 // ---------------------------------------------------------------- transpose
-// dst[h][c][perm(r)] = src[h][r][c] for r < rows, c < cols; dst row stride ld_dst >= rows
-// (a multiple of 16), the columns of r in rows..ld_dst-1 are zero filled.  perm swaps bits
+// dst[h][c][perm(r)] = src[h][r][c] for r < rows, c < cols, up to a multiple of 64 of r (zeros past the end): columns ld_dst
+// apart, their groups of 32 r ld_32 apart (32: one run per column; 32 * cols and ld_dst = 32: blocks of 32 r, all columns of
+// a block together, which a kernel that takes 32 r at a time reads in whole lines).  perm swaps bits
 // 2 and 3 of r: inside every group of 16 the order is 0-3, 8-11, 4-7, 12-15, which puts
 // the 8 rows a lane half needs as MFMA k-slots (4 g + 0..3 and 8 + 4 g + 0..3) side by
 // side, so that operand is ONE 16-byte LDS read.
@@ -141,7 +142,7 @@ __device__ __forceinline__ u32x4 scale_bf16x8(u32x4 raw, float c) {
 // lanes that share a column fill its 128-byte line in two store instructions).  cols a multiple of 8.
 __global__ __launch_bounds__(64) void transpose_bf16_kernel(
     const uint16_t* __restrict__ src, int64_t src_hs, int64_t src_ld, int rows, int cols,
-    uint16_t* __restrict__ dst, int64_t dst_hs, int64_t ld_dst) {
+    uint16_t* __restrict__ dst, int64_t dst_hs, int64_t ld_dst, int64_t ld_32) {
   const int h = blockIdx.z;
   const int lane = threadIdx.x;
   const int rb = lane >> 3, cb = lane & 7;
@@ -155,8 +156,8 @@ __global__ __launch_bounds__(64) void transpose_bf16_kernel(
     in[j] = (r0 + j < rows) ? *reinterpret_cast<const u32x4*>(s + (int64_t)(r0 + j) * src_ld) : z;
   }
   // where the block's two halves go: r0 % 16 == 0 -> r0 and r0 + 8, r0 % 16 == 8 -> r0 - 4 and r0 + 4
-  const int p_lo = (r0 & 8) ? r0 - 4 : r0, p_hi = (r0 & 8) ? r0 + 4 : r0 + 8;
-  uint16_t* d = dst + (int64_t)h * dst_hs + (int64_t)c0 * ld_dst;
+  const int p_lo = ((r0 & 8) ? r0 - 4 : r0) & 31, p_hi = ((r0 & 8) ? r0 + 4 : r0 + 8) & 31;
+  uint16_t* d = dst + (int64_t)h * dst_hs + (int64_t)c0 * ld_dst + (r0 >> 5) * ld_32;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     // column c0 + i of the block: element e = in[e] element i
@@ -267,6 +268,44 @@ __device__ __forceinline__ void pin_block(f32x16& a) {
   asm volatile("" : "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15]));
 }
 
+// f(integral_constant<int, B>) .. f(integral_constant<int, E - 1>): a loop that is unrolled whatever its size
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
+// The 32 x 32 x 16 product of a kernel of one wave per SIMD (512 registers, half of them accumulation registers, which only
+// matrix instructions and loads can use).  The builtin's results lie in accumulation registers there, and every score costs a
+// move in and a move out.  Here the results lie in ordinary registers and the operands that no vector instruction
+// touches (A: just read from LDS; B of the score products: the queries) in the others.  The compiler does not see that an asm
+// statement is a matrix instruction: whoever reads a result keeps twelve issue slots clear of the last product on
+// it (three products behind it do: each takes the pipe for eight), and four between writing an operand and the product.
+#if SPX_MFMA_BUILTIN
+__device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) { d = mfma32(a, b, c); }
+__device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) { d = mfma32(a, b, d); }
+__device__ __forceinline__ void mfma32_onto_v(f32x16& d, bf16x8 a, bf16x8 b) { d = mfma32(a, b, d); }
+#else
+__device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+}
+__device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "a"(b));
+}
+__device__ __forceinline__ void mfma32_onto_v(f32x16& d, bf16x8 a, bf16x8 b) {  // B in ordinary registers
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
+}
+#endif
+// every product under way has arrived
+template <int N>
+__device__ __forceinline__ void mfma32_drain(f32x16 (&d)[N]) {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(d[i]));
+}
+
 // ---------------------------------------------------------------- forward
 // One workgroup = 4 waves = 4 * 32 * NSB query rows of one head (NSB = 2: a wave owns two 32-row
 // sub-blocks and every K / V^T fragment read from LDS feeds two MFMAs; the kernels run NSB = 1).
@@ -298,7 +337,7 @@ struct PrioPair {
 // buffers: a 16-byte LDS write from registers holds the LDS pipe twice as long as a 16-byte read, and these kernels keep
 // that pipe busy all the time.  The transposed operand of the second product comes out of the row-major tile through
 // transposing LDS reads (dQ: K^T; forward, TR: V^T), or, in larger forward calls, out of a copy V^T made once per call: two
-// 8-byte reads for one of 16 cost the forward 6 % at head_dim 128 and 20 % at 256, the copy is a launch of 4 us (fwd_tr).
+// 8-byte reads for one of 16 cost the forward 5 - 6 %, the copy is a launch of 4 us (fwd_tr).
 template <int D, int NW>
 struct FwdSmem {
   static constexpr int kTile = kBN * D * 2;  // unpadded, swizzled
@@ -397,8 +436,9 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
                         : make_rsrc(Vth, (uint32_t)((int64_t)D * p.NKVp * 2));
   constexpr int LPV = (D * 128 / 1024) / NW;             // V^T tile
   auto swz_vt = [](int r) { return (r >> 1) & 7; };
-  int k_row[TR ? 1 : LPK], k_col[TR ? 1 : LPK], v_off[TR ? 1 : LPV];
-  if constexpr (!TR) {
+  constexpr bool kWide = D > 128;  // one wave per SIMD: see wide_pass
+  int k_row[TR || kWide ? 1 : LPK], k_col[TR || kWide ? 1 : LPK], v_off[TR || kWide ? 1 : LPV];
+  if constexpr (!TR && !kWide) {
 #pragma unroll
     for (int j = 0; j < LPK; ++j) {
       const int r = (wave * LPK + j) * (1024 / RBK) + lane / CKK;
@@ -461,13 +501,10 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
   // The fragment reads as LDS addresses, one register per swizzle term, kept opaque to the
   // compiler: what is added to them per read (buffer, key half, 16-key step) is a constant and goes
   // into the offset field.  Formed on the symbol of the dynamic array instead, every read costs a
-  // vector add of that link-time constant.
-  // Only where both tile buffers lie inside the 64 KB an offset field reaches (head_dim <= 128); past
-  // that the constants need an add again and the registers are better left to the accumulators.
-  constexpr bool kAbsRd = 2 * SM::kBuf <= 65536;
+  // vector add of that link-time constant.  (Both tile buffers lie inside the 64 KB an offset field reaches.)
   const int rdv = col * 128 + ((g ^ swz_vt(col)) * 16);
-  uint32_t krd[kAbsRd ? NKK : 1], vrd0[kAbsRd && TR ? NDB : 1], vrd1[kAbsRd && TR ? NDB : 1], vrd[kAbsRd && !TR ? 4 : 1];
-  if constexpr (kAbsRd) {
+  uint32_t krd[NKK], vrd0[TR ? NDB : 1], vrd1[TR ? NDB : 1], vrd[TR ? 1 : 4];
+  if constexpr (!kWide) {
 #pragma unroll
     for (int j = 0; j < NKK; ++j) {
       krd[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
@@ -504,8 +541,6 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (n0 + kBN < blk_b) issue(n0 + kBN, buf ^ 1);
-      const uint8_t* const tk = fwd_smem + buf * SM::kBuf;
-      const uint8_t* const tv = tk + SM::kTile;
       if (n0 >= w_bmax || n0 + kBN <= w_amin) return;  // nothing visible for this wave
 
       f32x16 st[NSB][2];
@@ -518,11 +553,7 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
         constexpr int RG = SPX_FWD_RING;
         bf16x8 kfr[RG];
         auto kread = [&](int f) {
-          if constexpr (kAbsRd)
-            kfr[f % RG] = as_bf16x8(lds_read128(krd[f >> 1] + buf * SM::kBuf + (f & 1) * 32 * RBK));
-          else
-            kfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                tk + (f & 1) * 32 * RBK + (rdk ^ ((f >> 1) * 32))));
+          kfr[f % RG] = as_bf16x8(lds_read128(krd[f >> 1] + buf * SM::kBuf + (f & 1) * 32 * RBK));
         };
 #pragma unroll
         for (int f = 0; f < RG; ++f) kread(f);
@@ -606,21 +637,11 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
         bf16x8 vfr[RG];
         auto vread = [&](int f) {
           if constexpr (!TR) {
-            if constexpr (kAbsRd)
-              vfr[f % RG] = as_bf16x8(lds_read128(vrd[f / NDB] + buf * SM::kBuf + (f % NDB) * 32 * 128));
-            else
-              vfr[f % RG] = as_bf16x8(*reinterpret_cast<const u32x4*>(
-                  tv + (f % NDB) * 32 * 128 + (rdv ^ ((f / NDB) * 32))));
+            vfr[f % RG] = as_bf16x8(lds_read128(vrd[f / NDB] + buf * SM::kBuf + (f % NDB) * 32 * 128));
             return;
           }
-          i16x4 lo, hi;
-          if constexpr (kAbsRd) {
-            lo = lds_tr16(vrd0[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
-            hi = lds_tr16(vrd1[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
-          } else {
-            lo = lds_read_tr16(tv + (f / NDB) * 16 * RBK + (rt0 ^ ((f % NDB) * 64)));
-            hi = lds_read_tr16(tv + (f / NDB) * 16 * RBK + (rt1 ^ ((f % NDB) * 64)));
-          }
+          const i16x4 lo = lds_tr16(vrd0[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
+          const i16x4 hi = lds_tr16(vrd1[f % NDB] + buf * SM::kBuf + (f / NDB) * 16 * RBK);
           vfr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         };
 #pragma unroll
@@ -649,9 +670,310 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
     }
   };
 
-  run_pass(rb.a1, rb.b1, rb.w_a1min, rb.w_a1max, rb.w_b1min, rb.w_b1max, rb.blk_a1, rb.blk_b1);
-  if (p.a2)
-    run_pass(rb.a2, rb.b2, rb.w_a2min, rb.w_a2max, rb.w_b2min, rb.w_b2max, rb.blk_a2, rb.blk_b2);
+  // head_dim 256: the accumulators leave one wave per SIMD, so whatever this wave waits for its matrix pipe waits for too, and
+  // every other instruction has to be issued while a product runs (32 cycles each).  A tile is one unbroken row of 64 products
+  // in four quarters, each with a share of the rest beside it:
+  //   S0  scores of keys 0 - 31               second half of the soft-max of the last tile's keys 32 - 63; loads of K
+  //   O1  O += V^T P, LAST tile's keys 32 - 63   first half of the soft-max of keys 0 - 31; loads of V
+  //   S1  scores of keys 32 - 63              second half of the soft-max of keys 0 - 31
+  //   O0  O += V^T P, keys 0 - 31             first half of the soft-max of keys 32 - 63; the one barrier of the tile, four
+  //                                           products from the end, and the next tile's first reads behind it
+  // Operand fragments run sixteen products ahead through one ring.  V lies in LDS in halves of 32 keys, a ring of four: the second
+  // half of a tile is used, and so loaded, one tile late.  Soft-max reference and masking as in run_pass, per half.
+  // 16384 causal rows, 16 heads of 256, two K/V heads: 2375 us in the form of the other head sizes (all scores, the whole
+  // soft-max, all of O: matrix pipe busy 38 % of the cycles at 2.0 GHz, 176 moves between the register files per tile), 1800
+  // like this (62 % at 1.7 GHz: at the power limit); 600 rows 32.0 and 23.0.  The soft-max inside its own tile (two quarters
+  // without it, two with all of it) 1946; a ring of eight operands instead of sixteen 1 % more; V^T out of rows of the whole
+  // length, 64 bytes per load and row, in the place of blocks of 32 keys 12 % more.
+  auto wide_pass = [&](int a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
+    static_assert(NSB == 1, "one 32-row block per wave");
+    if (blk_b <= blk_a) return;
+    constexpr int RG = 16;
+    constexpr uint32_t kVoff = 2 * SM::kTile, kHalf = SM::kTile / 2;
+    int n0 = (blk_a / kBN) * kBN;
+    uint32_t par = 0;  // K buffer and pair of V halves of tile n0: 0 or kTile
+    // The lane's places in the first load of K and V; a later load of the tile is an XOR and an immediate away.  Rows past the
+    // end come in as zeros (they are masked out).  Formed for every tile: kept over the loop they would not leave room for the
+    // operands.
+    struct Places { int k, v; };
+    auto places = [&]() __attribute__((always_inline)) {
+      int at = lane;
+      asm volatile("" : "+v"(at));
+      const int b5 = at >> 5;
+      Places pl;
+      pl.k = (wave * 16 + b5) * RBK + ((at & 31) ^ b5) * 16;
+      pl.v = TR ? (wave * 8 + b5) * RBK + ((at & 31) ^ (b5 << 2) ^ ((wave & 1) << 1)) * 16
+                : wave * 4096 + (at >> 2) * 64 + ((at & 3) ^ ((at >> 4) & 3)) * 16;
+      return pl;
+    };
+    // load j (0 .. 7) of a wave's share of K tile n, load j (0 .. 3) of half h of V tile n
+    auto issue_k = [&](const Places& pl, int n, uint32_t to, auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+      const u32x4 res = make_rsrc(Kh + (int64_t)n * D, (uint32_t)(p.NKV - n) * RBK);
+      load_to_lds16<(j & 3) * 1024>(res, lds0 + to + wave * 8192 + (j >> 2) * 4096, pl.k ^ (32 * j | (j >> 2) << 12), 0);
+    };
+    auto issue_v = [&](const Places& pl, int n, int h2, uint32_t to, auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+      const uint32_t dst = lds0 + kVoff + to + h2 * kHalf + wave * 4096;
+      if constexpr (TR) {
+        const int row = min(n + 32 * h2, p.NKV);
+        const u32x4 res = make_rsrc(Vh + (int64_t)row * D, (uint32_t)(p.NKV - row) * RBK);
+        load_to_lds16<j * 1024>(res, dst, pl.v ^ (((j & 1) << 7) | ((j >> 1) << 4)), 0);
+      } else {
+        load_to_lds16<j * 1024>(vres, dst, pl.v, (n + 32 * h2) * (D * 2));  // (blocks of 32 keys: transpose_bf16_kernel)
+      }
+    };
+    // the sixteen loads of a tile: K and the first half of V of tile n1, the second half of tile n0
+    auto issue = [&](const Places& pl, int n1, auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+      if constexpr (j < 8) issue_k(pl, n1, SM::kTile - par, jc);
+      else if constexpr (j < 12) issue_v(pl, n1, 0, SM::kTile - par, std::integral_constant<int, j - 8>{});
+      else issue_v(pl, n0, 1, par, std::integral_constant<int, j - 12>{});
+    };
+
+    // fragment addresses, one register per swizzle term; the rest is in the offset field.  kr: K buffer of tile n0; vr0, vr1: V
+    // halves of the last tile until S1, then of this one
+    uint32_t kr[8], vr0[TR ? 4 : 2], vr1[TR ? 4 : 1];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) kr[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
+    if constexpr (TR) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        vr0[j] = lds0 + kVoff + SM::kTile + (uint32_t)(rt0 ^ (j * 64));
+        vr1[j] = lds0 + kVoff + SM::kTile + (uint32_t)(rt1 ^ (j * 64));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        vr0[j] = lds0 + kVoff + SM::kTile + (uint32_t)(col * 64 + (((g + 2 * j) ^ ((col >> 2) & 3)) * 16));
+    }
+    bf16x8 fr[RG];
+    auto fread = [&](auto fc) __attribute__((always_inline)) {
+      constexpr int f = decltype(fc)::value;
+      if constexpr ((f & 16) == 0) {
+        constexpr int kk = f & 15;
+        fr[f % RG] = as_bf16x8(lds_read128(kr[kk & 7] + (f >> 5) * 32 * RBK + (kk >> 3) * 256));
+      } else {
+        constexpr int h2 = f < 32, s = (f >> 3) & 1, db = f & 7;
+        if constexpr (!TR) {
+          fr[f % RG] = as_bf16x8(lds_read128(vr0[s] + h2 * kHalf + db * 32 * 64));
+        } else {
+          const i16x4 lo = lds_tr16(vr0[db & 3] + h2 * kHalf + s * 16 * RBK + (db >> 2) * 256);
+          const i16x4 hi = lds_tr16(vr1[db & 3] + h2 * kHalf + s * 16 * RBK + (db >> 2) * 256);
+          fr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+      }
+    };
+
+    f32x16 st[2];
+    u32x4 pb[2][2];
+    bf16x8 qa[NKK];
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+      qa[kk] = qf[0][kk];
+      asm volatile("" : "+a"(qa[kk]));  // (else a copy of them lives in ordinary registers and moves over for every tile)
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[1][r] = 0.f;
+    float mx = 0.f, rs = 0.f;
+    float slack = m_ref[0] == -INFINITY ? -INFINITY : kRefSlack;  // a row without a reference takes its first one
+    bool need_mask = false;
+    auto slots = [] { __builtin_amdgcn_sched_barrier(0); };
+    // the soft-max of one half in 32 pieces, one beside each product of two quarters; its scores are complete from piece 3 on
+    auto soft = [&](auto half_c, auto piece_c) __attribute__((always_inline)) {
+      constexpr int h2 = decltype(half_c)::value, pc = decltype(piece_c)::value;
+      f32x16& s = st[h2];
+      if constexpr (pc == 3) {
+        asm volatile("" : "+v"(s));
+        if (need_mask) {
+          const int m_lo = a_i - n0 - 4 * g, m_hi = b_i - n0 - 4 * g;
+          asm volatile("" : "+v"(s));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int cr = h2 * 32 + 8 * (r >> 2) + (r & 3);
+            if (cr < m_lo || cr >= m_hi) s[r] = -INFINITY;
+          }
+          asm volatile("" : "+v"(s));
+        }
+        mx = fmaxf(s[0], s[1]);
+#pragma unroll
+        for (int r = 2; r < 8; r += 2) mx = fmaxf(fmaxf(mx, s[r]), s[r + 1]);
+      } else if constexpr (pc == 4) {
+#pragma unroll
+        for (int r = 8; r < 16; r += 2) mx = fmaxf(fmaxf(mx, s[r]), s[r + 1]);
+      } else if constexpr (pc == 5) {
+        mx = half_swap_max(mx);
+      } else if constexpr (pc == 6) {
+        const bool move = mx > slack;
+        if (__builtin_amdgcn_ballot_w64(move) != 0) {
+          // some row's reference moves: its sum, what O has taken so far, and the probabilities of the half whose products
+          // are under way
+          mfma32_drain(st);
+          mfma32_drain(acc[0]);
+          const bool unset = m_ref[0] == -INFINITY;
+          const float delta = move ? mx : 0.f;
+          const float alpha = (move && !unset) ? fast_exp2(-delta) : 1.f;  // unset rows hold zeros
+          m_ref[0] = move ? (unset ? mx : m_ref[0] + mx) : m_ref[0];
+          slack = move ? kRefSlack : slack;
+          const float nr = unset && !move ? 0.f : -m_ref[0];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            nref[0][r] = nr;
+            s[r] -= delta;
+            st[1 - h2][r] *= alpha;
+          }
+          pb[1 - h2][0] = __builtin_bit_cast(u32x4, pack8(st[1 - h2], 0));
+          pb[1 - h2][1] = __builtin_bit_cast(u32x4, pack8(st[1 - h2], 8));
+          l_run[0] *= alpha;
+#pragma unroll
+          for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][db][r] *= alpha;
+          mfma32_drain(st);
+          mfma32_drain(acc[0]);
+        }
+        rs = 0.f;
+      } else if constexpr (pc >= 7 && pc < 23) {
+        s[pc - 7] = fast_exp2(s[pc - 7]);
+        rs += s[pc - 7];
+      } else if constexpr (pc >= 23 && pc < 31) {
+        constexpr int w = pc - 23;
+        pb[h2][w >> 2][w & 3] = pack_bf16x2(s[2 * w], s[2 * w + 1]);
+      } else if constexpr (pc == 31) {
+        l_run[0] += rs;
+      }
+    };
+
+    // everybody's reads of this tile are done and the next one has landed: over to its buffers
+    auto next_tile = [&]() __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __syncthreads();
+      const uint32_t d = SM::kTile - 2 * par;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) kr[j] += d;
+      par = SM::kTile - par;
+      n0 = __builtin_amdgcn_readfirstlane(n0 + kBN);
+    };
+    // the V addresses from tile n0 - 64 to tile n0 (first: whatever they are at, to n0)
+    auto next_v = [&]() __attribute__((always_inline)) {
+      const uint32_t d = 2 * par - SM::kTile;
+#pragma unroll
+      for (int j = 0; j < (TR ? 4 : 2); ++j) {
+        vr0[j] += d;
+        if constexpr (TR) vr1[j] += d;
+      }
+    };
+    // (past the last tile: this one's loads again, nobody reads them)
+    auto ahead = [&]() __attribute__((always_inline)) { return n0 + kBN < blk_b ? n0 + kBN : n0; };
+    // tiles that this wave sees nothing of (a run at either end): its share of the loads
+    auto skip_to = [&](int stop) __attribute__((always_inline)) {
+#pragma unroll 1
+      while (n0 < stop) {
+        const int n1 = ahead();
+        const Places pl = places();
+        static_for<0, 16>([&](auto j) __attribute__((always_inline)) { issue(pl, n1, j); });
+        next_tile();
+      }
+    };
+    auto tile = [&](auto first_c) __attribute__((always_inline)) {
+      constexpr bool first = decltype(first_c)::value;
+      const int n1 = ahead();
+      const Places pl = places();
+      static_for<0, 16>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        slots();
+        if constexpr (f == 0) mfma32_from(st[0], fr[f % RG], qa[f], nref[0]);
+        else mfma32_onto(st[0], fr[f % RG], qa[f]);
+        slots();
+        fread(std::integral_constant<int, f + RG + (first ? 16 : 0)>{});
+        if constexpr (!first) soft(std::integral_constant<int, 1>{}, std::integral_constant<int, 16 + f>{});
+        if constexpr (f % 2 == 0) issue(pl, n1, std::integral_constant<int, f / 2>{});
+      });
+      need_mask = (n0 < w_amax) || (n0 + kBN > w_bmin);
+      if constexpr (first) mfma32_drain(st);
+      static_for<0, 16>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        if constexpr (!first) {
+          slots();
+          mfma32_onto_v(acc[0][f & 7], fr[f % RG], as_bf16x8(pb[1][f >> 3]));
+          slots();
+          fread(std::integral_constant<int, 16 + f + RG>{});
+        }
+        soft(std::integral_constant<int, 0>{}, fc);
+        if constexpr (f % 2 == 0) issue(pl, n1, std::integral_constant<int, 8 + f / 2>{});
+      });
+      slots();
+      next_v();
+      static_for<0, 16>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        slots();
+        if constexpr (f == 0) mfma32_from(st[1], fr[f % RG], qa[f], nref[0]);
+        else mfma32_onto(st[1], fr[f % RG], qa[f]);
+        slots();
+        fread(std::integral_constant<int, 32 + f + RG>{});
+        soft(std::integral_constant<int, 0>{}, std::integral_constant<int, 16 + f>{});
+      });
+      static_for<0, 16>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        slots();
+        mfma32_onto_v(acc[0][f & 7], fr[f % RG], as_bf16x8(pb[0][f >> 3]));
+        slots();
+        soft(std::integral_constant<int, 1>{}, fc);
+        if constexpr (f == 8) next_tile();
+        if constexpr (f >= 8) {
+          fread(std::integral_constant<int, 2 * f - 16>{});
+          fread(std::integral_constant<int, 2 * f - 15>{});
+        }
+      });
+      slots();
+    };
+
+    __syncthreads();  // a previous pass may still be reading its buffers
+    {
+      const Places pl = places();
+      static_for<0, 8>([&](auto j) __attribute__((always_inline)) { issue_k(pl, n0, 0, j); });
+      static_for<0, 4>([&](auto j) __attribute__((always_inline)) { issue_v(pl, n0, 0, 0, j); });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    skip_to(min(w_amin - kBN + 1, blk_b));
+    const int seen = min(w_bmax, blk_b);
+    if (n0 < seen) {
+#pragma unroll
+      for (int j = 0; j < (TR ? 4 : 2); ++j) {  // where the tile before the first one would lie
+        vr0[j] -= par;
+        if constexpr (TR) vr1[j] -= par;
+      }
+      static_for<0, RG>([&](auto f) __attribute__((always_inline)) { fread(f); });
+      tile(std::true_type{});
+#pragma unroll 1
+      while (n0 < seen) tile(std::false_type{});
+      // the last tile's keys 32 - 63
+      mfma32_drain(st);
+      static_for<16, 32>([&](auto pc) __attribute__((always_inline)) { soft(std::integral_constant<int, 1>{}, pc); });
+      static_for<16, 16 + RG>([&](auto f) __attribute__((always_inline)) { fread(f); });
+      static_for<0, 16>([&](auto fc) __attribute__((always_inline)) {
+        constexpr int f = decltype(fc)::value;
+        slots();
+        mfma32_onto_v(acc[0][f & 7], fr[f % RG], as_bf16x8(pb[1][f >> 3]));
+        slots();
+      });
+      mfma32_drain(acc[0]);
+    }
+    skip_to(blk_b);
+  };
+
+  if constexpr (kWide) {
+#pragma unroll 1
+    for (int c = 0; c < (p.a2 ? 2 : 1); ++c)  // (one copy of the code for both interval classes)
+      wide_pass(c ? rb.a2[0] : rb.a1[0], c ? rb.b2[0] : rb.b1[0], c ? rb.w_a2min : rb.w_a1min, c ? rb.w_a2max : rb.w_a1max,
+                c ? rb.w_b2min : rb.w_b1min, c ? rb.w_b2max : rb.w_b1max, c ? rb.blk_a2 : rb.blk_a1,
+                c ? rb.blk_b2 : rb.blk_b1);
+  } else {
+    run_pass(rb.a1, rb.b1, rb.w_a1min, rb.w_a1max, rb.w_b1min, rb.w_b1max, rb.blk_a1, rb.blk_b1);
+    if (p.a2)
+      run_pass(rb.a2, rb.b2, rb.w_a2min, rb.w_a2max, rb.w_b2min, rb.w_b2max, rb.blk_a2, rb.blk_b2);
+  }
 
   // from here on l_run is the whole row's sum in both lanes of a query
 #pragma unroll
@@ -1313,11 +1635,12 @@ static DkvPlan dkv_plan(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
 }
 
 // Forward calls of little work take V^T from transposing reads, larger ones from a copy: the copy pays above about 60 us of
-// products at head_dim <= 128 and 16 us at 256 (at 800 TFLOP/s of a causal mask).  Measured, copy + kernel against
-// transposing reads: 512 rows, 32 heads of 64 16.9 / 13.4 us, 2048 of 128 57.7 / 58.3, 4096 of 128 145 / 147, 16384 rows of
-// 16 heads of 256 2485 / 3072.
+// products at head_dim <= 128 and 1000 us at 256 (at 800 TFLOP/s of a causal mask).  Measured, copy + kernel against
+// transposing reads: 512 rows, 32 heads of 64 16.9 / 13.4 us, 2048 of 128 57.7 / 58.3, 4096 of 128 145 / 147; 600 rows of
+// 16 heads of 256 26.4 / 24.1, 2000 60.8 / 58.2, 4096 140.2 / 137.9, 8192 489 / 487, 16384 1835 / 1853 (two documents of 16380
+// after a second of work, at a lower clock: 3837 / 3860).
 static double fwd_us(int64_t NQ, int64_t NKV, int Hq, int D) { return 2. * Hq * (double)NQ * (double)NKV * D / 8e8; }
-static bool fwd_tr(int64_t NQ, int64_t NKV, int Hq, int D) { return fwd_us(NQ, NKV, Hq, D) < (D > 128 ? 16. : 60.); }
+static bool fwd_tr(int64_t NQ, int64_t NKV, int Hq, int D) { return fwd_us(NQ, NKV, Hq, D) < (D > 128 ? 1000. : 60.); }
 static int64_t fwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
   return fwd_tr(NQ, NKV, Hq, D) ? 256 : round_up((int64_t)Hkv * D * round_up(NKV, 128) * 2, 256);
 }
@@ -1361,7 +1684,8 @@ static int launch_fwd(AttnParams p, void* workspace, uint16_t* O, float* lse, hi
   uint16_t* vt = reinterpret_cast<uint16_t*>(workspace);
   dim3 tgrid((unsigned)(p.NKVp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hkv);
   hipLaunchKernelGGL(transpose_bf16_kernel, tgrid, dim3(64), 0, st, p.V, p.v_hs, (int64_t)D, p.NKV, D,
-                     vt, (int64_t)D * p.NKVp, (int64_t)p.NKVp);
+                     vt, (int64_t)D * p.NKVp, D > 128 ? (int64_t)32 : (int64_t)p.NKVp,
+                     D > 128 ? (int64_t)32 * D : (int64_t)32);
   return launch_fwd_as<D, false>(p, vt, O, lse, st, fn);
 }
 
@@ -1665,12 +1989,10 @@ extern "C" int spx_span_attn_bwd(const void* q, int64_t q_head_stride, const voi
 
 // ---------------------------------------------------------------- allocation-free variant
 // V^T of a large call lies in a device array of the library.  Transposing reads throughout need no array and take 3 - 5 %
-// longer at head_dim 128 and up to 10 % at 256: 8192 rows, 64 / 8 heads of 128 1003 us, from the copy 957; 16384 rows,
-// 16 / 2 heads of 256 2628 / 2386.  The array serves one call at a time: a call waits, on the device, for the event behind
-// the last one's kernels, whichever stream and host thread that came from.  A call under capture takes transposing reads:
-// nothing would order its replays.  The wait and the record cost 3 us, so the copy begins later here than in fwd_tr, at
-// 120 us of products (2048 rows, 16 heads of 256, 43 us: 89.5 us without the array, 92.3 with it; 4096 rows of 16 / 2
-// heads, 172 us: 187.3 / 178.5; 4096 rows, 32 heads of 128: 140.4 / 140.3).
+// longer: 8192 rows, 64 / 8 heads of 128 1003 us, from the copy 957.  The array serves one call at a time: a call waits, on
+// the device, for the event behind the last one's kernels, whichever stream and host thread that came from.  A call under
+// capture takes transposing reads: nothing would order its replays.  The wait and the record cost 3 us, so the copy begins
+// later here than in fwd_tr, at 120 us of products (4096 rows, 32 heads of 128: 140.4 us without the array, 140.3 with it).
 constexpr int64_t kStaticScratchBytes = 16ll << 20;
 constexpr double kStaticCopyUs = 120.;
 static __device__ __align__(256) unsigned char static_scratch[kStaticScratchBytes];
@@ -1726,7 +2048,7 @@ extern "C" int spx_ttt_attn_fwd_static(const void* q, int64_t q_head_stride, con
   if ((int64_t)Hkv * D * round_up(T, 128) * 2 > kStaticScratchBytes)
     return fail_arg(fname, "Hkv * D * round_up(T, 128) * 2 bytes exceed 16 MiB, the limit of this entry point; "
                            "use spx_ttt_attn_fwd with a caller-owned workspace");
-  const bool copies = fwd_us(T, T, Hq, D) >= kStaticCopyUs;
+  const bool copies = !fwd_tr(T, T, Hq, D) && fwd_us(T, T, Hq, D) >= kStaticCopyUs;
   return with_static_scratch(fname, copies, reinterpret_cast<hipStream_t>(stream), [&](void* workspace) {
     if (int rc = ttt_attn_fwd_impl(fname, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq, Hkv,
                                    D, scaling, out, lse, workspace, stream))
