@@ -1179,7 +1179,8 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
   const int qb = n_qb - 1 - rest / group;
   const int m0 = qb * BM;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, col = lane & 31;
   int i[NSB], ic[NSB];
   float lse_i[NSB], delta_i[NSB];
@@ -1295,7 +1296,7 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb) {
         // the 32-key halves of the tile one after the other: 32 score registers live
-#pragma unroll(D > 128 ? 1 : TB / 32)
+#pragma unroll
         for (int kb = 0; kb < TB / 32; ++kb) {
           f32x16 st, dp;
           // K and V fragments alternate through a ring of four registers (fragment 2 kk is
@@ -1366,9 +1367,167 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
     }
   };
 
-  run_pass(rb.a1, rb.b1, rb.w_a1min, rb.w_a1max, rb.w_b1min, rb.w_b1max, rb.blk_a1, rb.blk_b1);
-  if (p.a2)
-    run_pass(rb.a2, rb.b2, rb.w_a2min, rb.w_a2max, rb.w_b2min, rb.w_b2max, rb.blk_a2, rb.blk_b2);
+  // head_dim 256, one wave per SIMD (see the forward's wide_pass): the 96 products of a tile in one row, six sixths,
+  //   S0, dP0, S1, dP1   scores and dP of keys 0 - 31 and 32 - 63
+  //   O0, O1             dQ += K^T dS of the two halves
+  // with the tile's loads beside the first two, the exponentials of a half beside its dP, its dS beside the sixth after that,
+  // and the barrier and the next tile's first reads beside O1.
+  // 16384 causal rows, 16 heads, two K/V heads: 3350 us in the form of the other head sizes (matrix pipe busy 48 % at 1.95 GHz,
+  // 64 moves between the register files per half tile), 2520 like this (78 % at 1.6 GHz: at the power limit).
+  auto wide_pass = [&](int a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
+    static_assert(NSB == 1, "one 32-row block per wave");
+    if (blk_b <= blk_a) return;
+    constexpr int RG = 16;
+    int n0 = (blk_a / TB) * TB;
+    uint32_t buf = 0;
+    // the lane's place in the first load of a tile, formed for every tile; rows past the end come in as zeros (masked out)
+    auto place = [&]() __attribute__((always_inline)) {
+      int at = lane;
+      asm volatile("" : "+v"(at));
+      const int b5 = at >> 5;
+      return (wave * 16 + b5) * RBK + ((at & 31) ^ (b5 << 2)) * 16;
+    };
+    // load j of the wave's sixteen: rows of K, then of V
+    auto issue = [&](int pl, int n, uint32_t to, auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value & 7;
+      constexpr bool is_v = decltype(jc)::value >= 8;
+      const u32x4 res = make_rsrc((is_v ? Vh : Kh) + (int64_t)n * D, (uint32_t)(p.NKV - n) * RBK);
+      load_to_lds16<(j & 3) * 1024>(res, lds0 + to + (is_v ? SM::kTileK : 0) + wave * 8192 + (j >> 2) * 4096,
+                                    pl ^ (((j & 1) << 7) | ((j >> 1) & 3) << 4 | (j >> 2) << 12), 0);
+    };
+    // fragment addresses, one register per swizzle term: rows (K, V) and transposed (K)
+    uint32_t kr[8], tr0[4], tr1[4];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) kr[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      tr0[j] = lds0 + (uint32_t)(rt0 ^ (j * 64));
+      tr1[j] = lds0 + (uint32_t)(rt1 ^ (j * 64));
+    }
+    bf16x8 fr[RG];
+    auto fread = [&](auto fc) __attribute__((always_inline)) {
+      constexpr int f = decltype(fc)::value, i = f & 15;
+      if constexpr (f < 64) {  // K 0, V 0, K 1, V 1
+        fr[f % RG] = as_bf16x8(lds_read128(kr[i & 7] + ((f >> 4) & 1) * SM::kTileK + (f >> 5) * 32 * RBK + (i >> 3) * 256));
+      } else {
+        constexpr int off = ((f - 64) >> 4) * 32 * RBK + (i >> 3) * 16 * RBK + ((i >> 2) & 1) * 256;
+        const i16x4 lo = lds_tr16(tr0[i & 3] + off), hi = lds_tr16(tr1[i & 3] + off);
+        fr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+    };
+    f32x16 st[2], dp[2];
+    u32x4 ds[2][2];
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+a"(qf[0][kk]), "+a"(dof[0][kk]));
+    bool need_mask = false;
+    auto slots = [] { __builtin_amdgcn_sched_barrier(0); };
+    // p and dS of a half in 32 pieces from the first product of its dP on
+    auto soft = [&](auto half_c, auto piece_c) __attribute__((always_inline)) {
+      constexpr int h2 = decltype(half_c)::value, pc = decltype(piece_c)::value;
+      f32x16& s = st[h2];
+      if constexpr (pc == 3) asm volatile("" : "+v"(s));  // its last product is three behind
+      if constexpr (pc >= 3 && pc < 19) s[pc - 3] = fast_exp2(s[pc - 3]);
+      if constexpr (pc == 19) {
+        asm volatile("" : "+v"(dp[h2]));
+        if (need_mask) {
+          const int lo = a_i - n0 - 4 * g, hi = b_i - n0 - 4 * g;
+          asm volatile("" : "+v"(s));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int cr = h2 * 32 + 8 * (r >> 2) + (r & 3);
+            if (cr < lo || cr >= hi) s[r] = 0.f;
+          }
+          asm volatile("" : "+v"(s));
+        }
+      }
+      if constexpr (pc >= 20 && pc < 28) {
+        constexpr int w = pc - 20;
+        ds[h2][w >> 2][w & 3] = pack_bf16x2(dp[h2][2 * w] * s[2 * w], dp[h2][2 * w + 1] * s[2 * w + 1]);
+      }
+    };
+    auto next_tile = [&]() __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __syncthreads();
+      const uint32_t d = SM::kBuf - 2 * buf;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) kr[j] += d;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { tr0[j] += d; tr1[j] += d; }
+      buf = SM::kBuf - buf;
+      n0 = __builtin_amdgcn_readfirstlane(n0 + TB);
+    };
+    // (past the last tile: this one's loads again, nobody reads them)
+    auto ahead = [&]() __attribute__((always_inline)) { return n0 + TB < blk_b ? n0 + TB : n0; };
+    auto skip_to = [&](int stop) __attribute__((always_inline)) {
+#pragma unroll 1
+      while (n0 < stop) {
+        const int n1 = ahead(), pl = place();
+        static_for<0, 16>([&](auto j) __attribute__((always_inline)) { issue(pl, n1, SM::kBuf - buf, j); });
+        next_tile();
+      }
+    };
+    __syncthreads();  // a previous pass may still be reading its buffers
+    {
+      const int pl = place();
+      static_for<0, 16>([&](auto j) __attribute__((always_inline)) { issue(pl, n0, 0, j); });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    skip_to(min(w_amin - TB + 1, blk_b));
+    const int seen = min(w_bmax, blk_b);
+    if (n0 < seen) {
+      static_for<0, RG>([&](auto f) __attribute__((always_inline)) { fread(f); });
+#pragma unroll 1
+      do {
+        need_mask = (n0 < w_amax) || (n0 + TB > w_bmin);
+        const int n1 = ahead(), pl = place();
+        static_for<0, 96>([&](auto fc) __attribute__((always_inline)) {
+          constexpr int f = decltype(fc)::value, i = f & 15, part = f >> 4;
+          using I = std::integral_constant<int, i>;
+          using I16 = std::integral_constant<int, i + 16>;
+          using H0 = std::integral_constant<int, 0>;
+          using H1 = std::integral_constant<int, 1>;
+          slots();
+          if constexpr (part == 0 || part == 2) {
+            if constexpr (i == 0) mfma32_from(st[part >> 1], fr[f % RG], qf[0][i], nlse[0]);
+            else mfma32_onto(st[part >> 1], fr[f % RG], qf[0][i]);
+          } else if constexpr (part == 1 || part == 3) {
+            if constexpr (i == 0) mfma32_from(dp[part >> 1], fr[f % RG], dof[0][i], ndel[0]);
+            else mfma32_onto(dp[part >> 1], fr[f % RG], dof[0][i]);
+          } else {
+            mfma32_onto_v(acc[0][i & 7], fr[f % RG], as_bf16x8(ds[part - 4][i >> 3]));
+          }
+          slots();
+          if constexpr (f + RG < 96) fread(std::integral_constant<int, f + RG>{});
+          if constexpr (part == 1) soft(H0{}, I{});
+          if constexpr (part == 2) soft(H0{}, I16{});
+          if constexpr (part == 3) soft(H1{}, I{});
+          if constexpr (part == 4) soft(H1{}, I16{});
+          if constexpr (part < 2 && i % 2 == 0) issue(pl, n1, SM::kBuf - buf, std::integral_constant<int, part * 8 + i / 2>{});
+          if constexpr (f == 88) next_tile();
+          if constexpr (f >= 88) {
+            fread(std::integral_constant<int, 2 * (f - 88)>{});
+            fread(std::integral_constant<int, 2 * (f - 88) + 1>{});
+          }
+        });
+        slots();
+      } while (n0 < seen);
+      mfma32_drain(acc[0]);
+    }
+    skip_to(blk_b);
+  };
+
+  if constexpr (D > 128) {
+#pragma unroll 1
+    for (int c = 0; c < (p.a2 ? 2 : 1); ++c)  // (one copy of the code for both interval classes)
+      wide_pass(c ? rb.a2[0] : rb.a1[0], c ? rb.b2[0] : rb.b1[0], c ? rb.w_a2min : rb.w_a1min, c ? rb.w_a2max : rb.w_a1max,
+                c ? rb.w_b2min : rb.w_b1min, c ? rb.w_b2max : rb.w_b1max, c ? rb.blk_a2 : rb.blk_a1,
+                c ? rb.blk_b2 : rb.blk_b1);
+  } else {
+    run_pass(rb.a1, rb.b1, rb.w_a1min, rb.w_a1max, rb.w_b1min, rb.w_b1max, rb.blk_a1, rb.blk_b1);
+    if (p.a2)
+      run_pass(rb.a2, rb.b2, rb.w_a2min, rb.w_a2max, rb.w_b2min, rb.w_b2max, rb.blk_a2, rb.blk_b2);
+  }
 
   // TTT diagonal keys: the key / value rows of a wave's 32 queries come in as coalesced 1 KB wave
   // loads global -> LDS into the wave's share of the tile buffers (see the forward kernel)

@@ -1,7 +1,7 @@
-"""Attention at head_dim 256 (``attn_fwd_kernel``'s ``wide_pass``: 64 products in a row with the soft-max of each half tile spread
-beside them) against the explicit soft-max in float64 over the same rounded queries: odd row counts around the 32-key
-halves, 64-key tiles and 128-row workgroups, rows and whole tiles a wave sees nothing of, and scores whose maximum
-moves on in every half tile, in one jump, or never."""
+"""Attention at head_dim 256 (``wide_pass`` of ``attn_fwd_kernel`` and ``attn_bwd_dq_kernel``: the products of a tile in one row
+with everything else spread beside them) against the explicit soft-max in float64 over the same rounded queries: odd row
+counts around the 32-key halves, 64-key tiles and 128-row workgroups, rows and whole tiles a wave sees nothing of, and
+scores whose maximum moves on in every half tile, in one jump, or never."""
 
 import pytest
 import torch
@@ -10,14 +10,22 @@ pytestmark = pytest.mark.gpu
 LOG2E = 1.4426950408889634
 
 
-def _reference(q, k, v, dense, scale):
-    """float64 soft-max over bf16(q * scale * log2 e), which is what the kernel multiplies with the keys"""
-    q, k, v, dense = (x.cuda() for x in (q, k, v, dense))
+def _reference(q, k, v, dense, scale, go):
+    """``(out, dq, bound)`` by the float64 soft-max over bf16(q * scale * log2 e), which is what the kernels multiply with the
+    keys.  ``bound``: what dq may be off by, element by element -- dS and dq are rounded to bf16 (2^-9 each, and twice that
+    for the fp32 sums and the exponential of fp32 scores), and delta is taken with the rounded output."""
+    q, k, v, dense, go = (x.cuda() for x in (q, k, v, dense, go))
     qs = (q.float() * (torch.tensor(scale, dtype=torch.float32) * LOG2E)).bfloat16().double()
     group = q.shape[1] // k.shape[1]
     kk, vv = (x.double().repeat_interleave(group, 1) for x in (k, v))
-    s = (qs @ kk.transpose(-1, -2)).masked_fill(~dense, float("-inf"))
-    return (torch.softmax(s * 0.6931471805599453, -1) @ vv).transpose(1, 2).cpu()
+    p = torch.softmax((qs @ kk.transpose(-1, -2)).masked_fill(~dense, float("-inf")) * 0.6931471805599453, -1)
+    out = p @ vv
+    do = go.double().transpose(1, 2)
+    ds = p * (do @ vv.transpose(-1, -2) - (do * out).sum(-1, keepdim=True))
+    dq = scale * (ds @ kk)
+    d_delta = 2.0 ** -8 * (do.abs() * out.abs()).sum(-1, keepdim=True)
+    bound = scale * ((2.0 ** -7 * ds.abs() + d_delta * p) @ kk.abs()) + 2.0 ** -8 * dq.abs() + 1e-6
+    return out.transpose(1, 2).cpu(), dq.cpu(), bound.cpu()
 
 
 def _rows(t, hq, hkv, kind, steps=1):
@@ -36,10 +44,18 @@ def _rows(t, hq, hkv, kind, steps=1):
     return tuple(x.bfloat16() for x in (q, k, v))
 
 
-def _check(out, want, v):
+def _check(fn, q, k, v, mask, dense):
+    scale = 256 ** -0.5
+    go = torch.randn(1, q.shape[2], q.shape[1], 256, generator=torch.Generator().manual_seed(1)).bfloat16()
+    qg = q.cuda().requires_grad_(True)
+    out = fn(qg, k.cuda(), v.cuda(), mask, scale)
+    out.backward(go.cuda())
+    want, dq, bound = _reference(q, k, v, dense, scale, go)
     # bf16 probabilities and result: two roundings of 2^-9 of at most max |v|; the rest is fp32
-    err = (out.double().cpu() - want).abs().max().item()
+    err = (out.detach().double().cpu() - want).abs().max().item()
     assert torch.isfinite(out).all() and err <= 2.0 ** -7 * v.float().abs().max().item(), err
+    off = (qg.grad.double().cpu() - dq).abs()
+    assert torch.isfinite(qg.grad).all() and (off <= bound).all(), ((off - bound).max().item(), off.max().item())
 
 
 @pytest.mark.parametrize("kind", ["flat", "rise", "fall", "jump"])
@@ -53,8 +69,7 @@ def test_rows_and_reference_moves(t, window, docs, kind):
     doc = torch.arange(t) * docs // t
     q, k, v = _rows(t, hq, hkv, kind)
     mask = A.create_ttt_mask(doc.cuda(), t, window)
-    out = A.ttt_attention(q.cuda(), k.cuda(), v.cuda(), mask, 256 ** -0.5)
-    _check(out, _reference(q, k, v, OMK.ttt_mask_dense(doc, t, 0, window), 256 ** -0.5), v)
+    _check(A.ttt_attention, q, k, v, mask, OMK.ttt_mask_dense(doc, t, 0, window))
 
 
 @pytest.mark.parametrize("kind", ["flat", "rise"])
@@ -70,5 +85,4 @@ def test_two_intervals_per_row(t, window, kind):
     q, _, _ = _rows(nq, 4, 2, kind)
     _, k, v = _rows(t + nq, 4, 2, kind)
     mask = A.create_dflash_mask(doc.cuda(), t, anchors.cuda(), 8, window)
-    out = A.dflash_attention(q.cuda(), k.cuda(), v.cuda(), mask, 256 ** -0.5)
-    _check(out, _reference(q, k, v, OMK.dflash_mask_dense(doc, t, anchors, 8, window), 256 ** -0.5), v)
+    _check(A.dflash_attention, q, k, v, mask, OMK.dflash_mask_dense(doc, t, anchors, 8, window))
