@@ -540,6 +540,10 @@ int spx_rmsnorm_bwd_partial(const void* x, int64_t ld_x, const void* weight, con
                             int32_t accumulate, int64_t rows, int64_t H, void* stream);
 int spx_rmsnorm_dweight(const float* dw_scratch, int64_t slots, int64_t H, void* dweight,
                         void* stream);
+/* The same for count (1 .. 16) gains in one launch; dweight[i] is fp32 where is_f32[i].  The five arrays are host memory, read
+ * before the call returns. */
+int spx_rmsnorm_dweights(const float* const* dw_scratch, const int64_t* slots, const int64_t* H, void* const* dweight,
+                         const int32_t* is_f32, int32_t count, void* stream);
 
 /* Two RMSNorms of one row count in one launch, written into the halves of y [rows, 2H] (row stride ld_y):
  * y[:, :H] = norm(a), y[:, H:] = norm(b); rstd [2, rows].  The backward of both (dy as y; dres_b, may be null,

@@ -133,6 +133,7 @@ PyMethodDef g_methods[] = {
     SPX_HOST("loss_step", spx_layer_loss_step)
     SPX_HOST("loss_terms", spx_layer_loss_terms)
     SPX_HOST("cat_bf16", spx_layer_cat_bf16)
+    SPX_HOST("gain_sums", spx_layer_gain_sums)
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -3,6 +3,9 @@
 // call); from here it costs the launch, 3 to 4 us.  Up to a thousand tokens a draft's step was bound by that: 512 tokens of
 // the 1B shape, three TTT steps: 2.50 ms -> 2.36 a pass; three layers of anchored blocks over 1777: 3.76 -> 3.61.
 
+#include <algorithm>
+#include <vector>
+
 #include "host_common.h"
 
 namespace {
@@ -473,5 +476,41 @@ PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor out = at::empty(shape, first.options().dtype(at::kBFloat16).requires_grad(false));
   check(spx_cat_bf16(src, elements, f32, n, out.mutable_data_ptr(), stream_of(first)), "spx_cat_bf16");
   return wrapped(released, out);
+  END_HANDLE_TH_ERRORS
+}
+
+// (partial sums, slots, H, fp32 out?) per gain -> a tuple of their sums [H], sixteen gains to a launch
+PyObject* spx_layer_gain_sums(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n >= 4 && n % 4 == 0, "gain_sums takes four arguments for every gain");
+  const int64_t gains = n / 4;
+  Args x("gain_sums", args, n, n);
+  std::vector<Tensor> part(gains), out(gains);
+  std::vector<const float*> from(gains);
+  std::vector<void*> into(gains);
+  std::vector<int64_t> slots(gains), h(gains);
+  std::vector<int32_t> f32(gains);
+  for (int64_t i = 0; i < gains; ++i) {
+    part[i] = x.tensor();
+    slots[i] = x.integer();
+    h[i] = x.integer();
+    f32[i] = x.integer() != 0;
+    TORCH_CHECK_VALUE(part[i].scalar_type() == at::kFloat && part[i].is_contiguous() && slots[i] > 0 && h[i] > 0 &&
+                          part[i].numel() >= slots[i] * h[i] && part[i].device() == part[0].device(),
+                      "contiguous fp32 partial sums of slots x H, on one device");
+  }
+  Unlocked released;
+  for (int64_t i = 0; i < gains; ++i) {
+    out[i] = at::empty({h[i]}, part[i].options().dtype(f32[i] ? at::kFloat : at::kBFloat16).requires_grad(false));
+    from[i] = part[i].const_data_ptr<float>();
+    into[i] = out[i].mutable_data_ptr();
+  }
+  for (int64_t i = 0; i < gains; i += 16)
+    check(spx_rmsnorm_dweights(&from[i], &slots[i], &h[i], &into[i], &f32[i], (int32_t)std::min<int64_t>(16, gains - i),
+                               stream_of(part[0])), "spx_rmsnorm_dweights");
+  released.lock();
+  PyObject* const all = PyTuple_New(gains);
+  for (int64_t i = 0; i < gains; ++i) PyTuple_SET_ITEM(all, i, THPVariable_Wrap(out[i]));
+  return all;
   END_HANDLE_TH_ERRORS
 }

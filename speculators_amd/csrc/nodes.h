@@ -20,3 +20,4 @@ PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_gain_sums(PyObject*, PyObject* const* args, Py_ssize_t n);

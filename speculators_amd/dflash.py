@@ -195,6 +195,7 @@ class DFlashDraftModel(nn.Module):
         # lm_head and the loss as one autograd node while the head is frozen and the loss is a single
         # fused reduction (False: always two nodes)
         self.fuse_head_loss = True
+        self._norms = [m for m in self.modules() if isinstance(m, RMSNorm)]  # staged together (WeightStager.gains)
 
     @property
     def mask_token_id(self) -> int:
@@ -259,6 +260,7 @@ class DFlashDraftModel(nn.Module):
         t = hidden_states.shape[1]
         bs = self.block_size
         self._stager.begin()
+        self._stager.gains(self._norms)
         hidden_states = compute_input(hidden_states)
         verifier_last_hidden_states = compute_input(verifier_last_hidden_states)
         if position_ids is None:

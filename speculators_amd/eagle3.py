@@ -297,6 +297,7 @@ class Eagle3DraftModel(nn.Module):
         # ``last_logits`` (for parity checks; the reference returns no logits either)
         self.keep_logits = False
         self.last_logits: list = []
+        self._norms = [m for m in self.modules() if isinstance(m, RMSNorm)]  # staged together (WeightStager.gains)
 
     # ------------------------------------------------------------------ helpers
     def load_vocab_mappings(self, t2d, d2t):
@@ -350,6 +351,7 @@ class Eagle3DraftModel(nn.Module):
         device = hidden_states.device
         t = hidden_states.shape[1]
         self._stager.begin(uses=ttt_steps)
+        self._stager.gains(self._norms)
         hidden_states = compute_input(hidden_states)
         if verifier_last_hidden_states is not None:
             verifier_last_hidden_states = compute_input(verifier_last_hidden_states)
@@ -396,15 +398,17 @@ class Eagle3DraftModel(nn.Module):
         draft_tokens = []
         self.last_logits = []
         for step in range(ttt_steps):
-            # looked up without a graph whatever embed_requires_grad says, as the reference does
-            # (models/eagle3/core.py:270-271): the flag only marks the parameter as trainable
-            with torch.no_grad():
-                # (the looked-up rows are cast to bf16 before the norm either way)
-                table = self.embed_tokens.weight
-                if not table.requires_grad:
-                    table = self._stager.get(table).w  # frozen: its bf16 copy is made once and kept
-                embeds = F.embedding(ids[:, step:step + t], table)
-            y = (embeds.to(hidden.dtype), hidden)
+            # looked up once for all steps (a step's rows are a window of them), without a graph whatever
+            # embed_requires_grad says, as the reference does (models/eagle3/core.py:270-271): the flag only marks
+            # the parameter as trainable
+            if step == 0:
+                with torch.no_grad():
+                    # (the looked-up rows are cast to bf16 before the norm either way)
+                    table = self.embed_tokens.weight
+                    if not table.requires_grad:
+                        table = self._stager.get(table).w  # frozen: its bf16 copy is made once and kept
+                    embeds = F.embedding(ids, table).to(hidden.dtype)
+            y = (embeds[:, step:step + t], hidden)
             normed = None
             last = len(self.layers) - 1
             # (the positions of step j are position_ids + j; a length-dependent rope type looks at them)

@@ -62,7 +62,7 @@ class GainGrads:
     """The gradient of one RMSNorm gain over ALL of its uses in one backward pass (a draft layer's
     norms run once per TTT step): the uses leave their partial column sums in one fp32 buffer --
     the first writes it, the others add to it inside their kernels -- and the node that staged
-    the gain (``weights._StageGain``), which autograd runs after every use, reduces it once.
+    the gain (``weights._StageGains``), which autograd runs after every use, reduces it once.
     A staged gain carries its ``GainGrads`` as the attribute ``spx_gain_grads``."""
 
     def __init__(self):
@@ -92,15 +92,10 @@ class GainGrads:
         self.marked = True
         return _lib.zero(device, torch.bfloat16).expand(self.h)
 
-    def finish(self):
-        """The summed gradient (bf16 ``[H]``) of the uses recorded since the last call, or None."""
+    def take(self):
+        """``(scratch, slots, H)`` of the uses recorded since the last call, or None."""
         scratch, self.scratch, self.marked = self.scratch, None, False
-        if scratch is None:
-            return None
-        dw = torch.empty(self.h, device=scratch.device, dtype=torch.bfloat16)
-        _lib.call("spx_rmsnorm_dweight", scratch, self.slots, self.h, dw,
-                  _lib.stream_ptr(scratch.device))
-        return dw
+        return None if scratch is None else (scratch, self.slots, self.h)
 
 
 def _norm_backward(grads, need_dw, x, w, dy, dres, rstd, dx, rows, h, tgt=None):

@@ -203,6 +203,7 @@ class MTPDraftModel(nn.Module):
         # lm_head and the loss as one autograd node while the head is frozen (False: two nodes, logits
         # returned with their own gradient path as in the reference)
         self.fuse_head_loss = True
+        self._norms = [m for m in self.modules() if isinstance(m, RMSNorm)]  # staged together (WeightStager.gains)
 
     @property
     def layers(self) -> nn.ModuleList:
@@ -227,6 +228,7 @@ class MTPDraftModel(nn.Module):
                 loss_mask=None, step_weights=None, return_dict: bool = True, **_kwargs):
         cfg = self.config
         self._stager.begin(uses=cfg.num_speculative_steps)
+        self._stager.gains(self._norms)
         hidden_states = compute_input(hidden_states)
         input_ids = input_ids.long()
         device = input_ids.device

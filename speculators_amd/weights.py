@@ -330,28 +330,43 @@ class _Stage(torch.autograd.Function):
         return (None, *grads)
 
 
-class _StageGain(torch.autograd.Function):
-    """bf16 compute copy of an RMSNorm gain (``1 + p`` for the zero-centred form).  Its backward
-    adds what the uses left in the gain's ``GainGrads`` (reduced here, once) to whatever gradient
-    arrives the ordinary way, and casts to the parameter's dtype."""
+class _StageGains(torch.autograd.Function):
+    """bf16 compute copies of RMSNorm gains (``1 + p`` for the zero-centred form).  Its backward
+    adds what the uses left in each gain's ``GainGrads`` (reduced here, all of them in one launch) to whatever
+    gradient arrives the ordinary way, in the parameter's dtype."""
 
     @staticmethod
-    def forward(ctx, p, plus_one, grads):
-        ctx.grads, ctx.dtype = grads, p.dtype
+    def forward(ctx, plus_one, grads, *ps):
+        ctx.grads, ctx.dtypes = grads, [p.dtype for p in ps]
+        ctx.set_materialize_grads(False)
         if plus_one:
-            return (1.0 + p.detach().float()).to(torch.bfloat16)
-        return p.detach().to(torch.bfloat16)
+            return tuple((1.0 + p.detach().float()).to(torch.bfloat16) for p in ps)
+        out = [p.detach() if p.dtype == torch.bfloat16 else None for p in ps]
+        cast = [i for i, w in enumerate(out) if w is None]
+        for at in range(0, len(cast), 4):  # (four to a launch)
+            some = cast[at:at + 4]
+            joint = _cat_bf16([ps[i] for i in some])
+            for i, w in zip(some, joint.split([ps[i].shape[0] for i in some]), strict=True):
+                out[i] = w
+        return tuple(out)
 
     @staticmethod
-    def backward(ctx, g):
-        total = ctx.grads.finish()
-        if total is None:
-            out = g
-        elif g is None or g.stride(0) == 0:  # nothing but the empty marker arrived
-            out = total
-        else:
-            out = (total.float() + g.float())
-        return (out.to(ctx.dtype) if out is not None else None), None, None
+    def backward(ctx, *gs):
+        taken = [grads.take() for grads in ctx.grads]
+        # (where a gradient arrives the ordinary way too -- not just the empty marker -- the sum is formed in fp32)
+        extra = [g if g is not None and (t is None or g.stride(0) != 0) else None for g, t in zip(gs, taken, strict=True)]
+        args = []
+        for t, g, dt in zip(taken, extra, ctx.dtypes, strict=True):
+            if t is not None:
+                args += [*t, int(g is not None or dt == torch.float32)]
+        sums = iter(_lib.native().gain_sums(*args)) if args else iter(())
+        out = []
+        for t, g, dt in zip(taken, extra, ctx.dtypes, strict=True):
+            total = g if t is None else next(sums)
+            if t is not None and g is not None:
+                total = total + g.float()
+            out.append(None if total is None else total.to(dt))
+        return (None, None, *out)
 
 
 class WeightStager:
@@ -403,22 +418,38 @@ class WeightStager:
     def gain(self, p: torch.Tensor, plus_one: bool = False) -> torch.Tensor:
         """A small 1-D weight (an RMSNorm gain) in bf16 for the running forward.  ``plus_one``: the
         gain is ``1 + p`` (evaluated in fp32), the form of the Qwen3-Next norms.  A trainable gain
-        goes through one autograd node (``_StageGain``) and carries a ``fused_ops.GainGrads``: the
+        goes through an autograd node (``_StageGains``) and carries a ``fused_ops.GainGrads``: the
         norm kernels of all its uses leave their partial sums there, and the node reduces them
         once, after the last use's backward."""
-        key = ("gain", id(p), plus_one)
-        hit = self._fwd.get(key)
+        hit = self._fwd.get(("gain", id(p), plus_one))
         if hit is None:
             _check_param_dtype(p)
             if p.requires_grad and torch.is_grad_enabled():
-                from .fused_ops import GainGrads
-
-                grads = GainGrads()
-                hit = _StageGain.apply(p, plus_one, grads)
-                hit.spx_gain_grads = grads
-            elif plus_one:
+                return self._stage_gains([p], plus_one)[0]
+            if plus_one:
                 hit = (1.0 + p.float()).to(torch.bfloat16)
             else:
-                hit = p if p.dtype == torch.bfloat16 else p.to(torch.bfloat16)
-            self._fwd[key] = hit
+                hit = p if p.dtype == torch.bfloat16 else self.get(p).w  # (frozen: its copy is kept)
+            self._fwd["gain", id(p), plus_one] = hit
         return hit
+
+    def gains(self, norms):
+        """Stages the gains of these norms (modules with ``weight``) through one node where they train: one launch casts
+        them (four at a time) and one sums their gradients, where each alone takes three launches."""
+        if not torch.is_grad_enabled():
+            return
+        ps = {id(n.weight): n.weight for n in norms if n.weight.requires_grad and n.weight.is_cuda}.values()
+        autocast = _autocast_bf16()
+        ps = [p for p in ps if p.dtype == torch.bfloat16 or (autocast and p.dtype == torch.float32)]
+        if len(ps) > 1 and all(p.device == ps[0].device for p in ps):
+            self._stage_gains(ps, False)
+
+    def _stage_gains(self, ps, plus_one):
+        from .fused_ops import GainGrads
+
+        grads = [GainGrads() for _ in ps]
+        out = _StageGains.apply(plus_one, grads, *ps)
+        for p, w, g in zip(ps, out, grads, strict=True):
+            w.spx_gain_grads = g
+            self._fwd["gain", id(p), plus_one] = w
+        return out
