@@ -282,7 +282,8 @@ __device__ __forceinline__ void static_for(F&& f) {
 // move in and a move out.  Here the results lie in ordinary registers and the operands that no vector instruction
 // touches (A: just read from LDS; B of the score products: the queries) in the others.  The compiler does not see that an asm
 // statement is a matrix instruction: whoever reads a result keeps twelve issue slots clear of the last product on
-// it (three products behind it do: each takes the pipe for eight), and four between writing an operand and the product.
+// it (three products behind it do: each takes the pipe for eight).  Nor does it keep a vector instruction that writes an
+// operand two issue slots away from the product (mfma32_operand).
 #if SPX_MFMA_BUILTIN
 __device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) { d = mfma32(a, b, c); }
 __device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) { d = mfma32(a, b, d); }
@@ -298,6 +299,8 @@ __device__ __forceinline__ void mfma32_onto_v(f32x16& d, bf16x8 a, bf16x8 b) {  
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
 }
 #endif
+// a product's operand is complete: not to be formed any later, and two issue slots from here to the product
+__device__ __forceinline__ void mfma32_operand(u32x4& x) { asm volatile("s_nop 1" : "+v"(x)); }
 // every product under way has arrived
 template <int N>
 __device__ __forceinline__ void mfma32_drain(f32x16 (&d)[N]) {
@@ -824,6 +827,8 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
           }
           pb[1 - h2][0] = __builtin_bit_cast(u32x4, pack8(st[1 - h2], 0));
           pb[1 - h2][1] = __builtin_bit_cast(u32x4, pack8(st[1 - h2], 8));
+          mfma32_operand(pb[1 - h2][0]);
+          mfma32_operand(pb[1 - h2][1]);
           l_run[0] *= alpha;
 #pragma unroll
           for (int db = 0; db < NDB; ++db)
@@ -839,6 +844,7 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
       } else if constexpr (pc >= 23 && pc < 31) {
         constexpr int w = pc - 23;
         pb[h2][w >> 2][w & 3] = pack_bf16x2(s[2 * w], s[2 * w + 1]);
+        if constexpr ((w & 3) == 3) mfma32_operand(pb[h2][w >> 2]);
       } else if constexpr (pc == 31) {
         l_run[0] += rs;
       }
@@ -1443,6 +1449,7 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
       if constexpr (pc >= 20 && pc < 28) {
         constexpr int w = pc - 20;
         ds[h2][w >> 2][w & 3] = pack_bf16x2(dp[h2][2 * w] * s[2 * w], dp[h2][2 * w + 1] * s[2 * w + 1]);
+        if constexpr ((w & 3) == 3) mfma32_operand(ds[h2][w >> 2]);
       }
     };
     auto next_tile = [&]() __attribute__((always_inline)) {
