@@ -1158,7 +1158,9 @@ struct DqSmem {
   static constexpr int kTileK = kBN * D * 2;
   static constexpr int kBuf = 2 * kTileK;
   static constexpr int kDiag = NW * 2 * 32 * D * 2;  // K and V rows of 32 queries per wave (TTT diagonal keys)
-  static constexpr int kTiles = 2 * kBuf > kDiag ? 2 * kBuf : kDiag;
+  static constexpr bool kWide = D != 128;  // attn_bwd_dq_kernel's wide_pass
+  static constexpr int kStages = D == 64 ? 3 : 2;
+  static constexpr int kTiles = kStages * kBuf > kDiag ? kStages * kBuf : kDiag;
   static constexpr int kBytes = kTiles + 4 * NW * (int)sizeof(int);
 };
 
@@ -1373,51 +1375,59 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
     }
   };
 
-  // head_dim 256, one wave per SIMD (see the forward's wide_pass): the 96 products of a tile in one row, six sixths,
+  // head_dim 256 with one wave per SIMD (see the forward's wide_pass), 64 with two: the 6 * D / 16 products of a tile in one row,
+  // six sixths,
   //   S0, dP0, S1, dP1   scores and dP of keys 0 - 31 and 32 - 63
   //   O0, O1             dQ += K^T dS of the two halves
   // with the tile's loads beside the first two, the exponentials of a half beside its dP, its dS beside the sixth after that,
   // and the barrier and the next tile's first reads beside O1.
   // 16384 causal rows, 16 heads, two K/V heads: 3350 us in the form of the other head sizes (matrix pipe busy 48 % at 1.95 GHz,
-  // 64 moves between the register files per half tile), 2520 like this (78 % at 1.6 GHz: at the power limit).
+  // 64 moves between the register files per half tile), 2520 like this (78 % at 1.6 GHz: at the power limit).  32 heads of 64:
+  // 512 rows 15.7 and 14.7, 4096 125 and 114, 8192 under a window of 2048 209 and 196.  At head_dim 128 this needs more
+  // registers than two waves of a SIMD have, and with one wave a call of more than one workgroup per compute unit loses:
+  // 4096 rows of 32 heads 227 and 233, 8192 of 64 1370 and 1424 (1024 of 32: 32.2 and 27.8).
   auto wide_pass = [&](int a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
     static_assert(NSB == 1, "one 32-row block per wave");
     if (blk_b <= blk_a) return;
-    constexpr int RG = 16;
+    constexpr int RG = D > 64 ? 16 : 8, NS = SM::kStages;
+    constexpr int kLoads = 2 * LPK;                 // of a wave and tile: rows of K, then of V
+    constexpr int XRW = 1024 / RBK;                 // rows per load
     int n0 = (blk_a / TB) * TB;
     uint32_t buf = 0;
     // the lane's place in the first load of a tile, formed for every tile; rows past the end come in as zeros (masked out)
     auto place = [&]() __attribute__((always_inline)) {
       int at = lane;
       asm volatile("" : "+v"(at));
-      const int b5 = at >> 5;
-      return (wave * 16 + b5) * RBK + ((at & 31) ^ (b5 << 2)) * 16;
+      const int r = wave * (LPK * XRW) + at / CKK;
+      return r * RBK + ((at % CKK) ^ swz_k(r)) * 16;
     };
-    // load j of the wave's sixteen: rows of K, then of V
     auto issue = [&](int pl, int n, uint32_t to, auto jc) __attribute__((always_inline)) {
-      constexpr int j = decltype(jc)::value & 7;
-      constexpr bool is_v = decltype(jc)::value >= 8;
+      constexpr int j = decltype(jc)::value % LPK;
+      constexpr bool is_v = decltype(jc)::value >= LPK;
       const u32x4 res = make_rsrc((is_v ? Vh : Kh) + (int64_t)n * D, (uint32_t)(p.NKV - n) * RBK);
-      load_to_lds16<(j & 3) * 1024>(res, lds0 + to + (is_v ? SM::kTileK : 0) + wave * 8192 + (j >> 2) * 4096,
-                                    pl ^ (((j & 1) << 7) | ((j >> 1) & 3) << 4 | (j >> 2) << 12), 0);
+      // what the row j * XRW adds to the swizzle of the first load's row
+      constexpr int dsw = CKK == 8 ? ((j & 1) << 1) : CKK == 16 ? (j & 3) : ((j & 1) << 3) | ((j >> 1) & 3);
+      load_to_lds16<(j & 3) * 1024>(res, lds0 + to + (is_v ? SM::kTileK : 0) + wave * (LPK * 1024) + (j >> 2) * 4096,
+                                    pl ^ (dsw << 4 | (j >> 2) << 12), 0);
     };
     // fragment addresses, one register per swizzle term: rows (K, V) and transposed (K)
-    uint32_t kr[8], tr0[4], tr1[4];
+    constexpr int NR = NKK < 8 ? NKK : 8, NT = NDB < 4 ? NDB : 4;
+    uint32_t kr[NR], tr0[NT], tr1[NT];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) kr[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
+    for (int j = 0; j < NR; ++j) kr[j] = lds0 + (uint32_t)(rdk ^ (j * 32));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NT; ++j) {
       tr0[j] = lds0 + (uint32_t)(rt0 ^ (j * 64));
       tr1[j] = lds0 + (uint32_t)(rt1 ^ (j * 64));
     }
     bf16x8 fr[RG];
     auto fread = [&](auto fc) __attribute__((always_inline)) {
-      constexpr int f = decltype(fc)::value, i = f & 15;
-      if constexpr (f < 64) {  // K 0, V 0, K 1, V 1
-        fr[f % RG] = as_bf16x8(lds_read128(kr[i & 7] + ((f >> 4) & 1) * SM::kTileK + (f >> 5) * 32 * RBK + (i >> 3) * 256));
+      constexpr int f = decltype(fc)::value, part = f / NKK, i = f % NKK;
+      if constexpr (part < 4) {  // K 0, V 0, K 1, V 1
+        fr[f % RG] = as_bf16x8(lds_read128(kr[i % NR] + (part & 1) * SM::kTileK + (part >> 1) * 32 * RBK + (i / NR) * 256));
       } else {
-        constexpr int off = ((f - 64) >> 4) * 32 * RBK + (i >> 3) * 16 * RBK + ((i >> 2) & 1) * 256;
-        const i16x4 lo = lds_tr16(tr0[i & 3] + off), hi = lds_tr16(tr1[i & 3] + off);
+        constexpr int db = i % NDB, off = (part - 4) * 32 * RBK + (i / NDB) * 16 * RBK + (db / NT) * 256;
+        const i16x4 lo = lds_tr16(tr0[db % NT] + off), hi = lds_tr16(tr1[db % NT] + off);
         fr[f % RG] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
     };
@@ -1427,13 +1437,20 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
     for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+a"(qf[0][kk]), "+a"(dof[0][kk]));
     bool need_mask = false;
     auto slots = [] { __builtin_amdgcn_sched_barrier(0); };
-    // p and dS of a half in 32 pieces from the first product of its dP on
-    auto soft = [&](auto half_c, auto piece_c) __attribute__((always_inline)) {
-      constexpr int h2 = decltype(half_c)::value, pc = decltype(piece_c)::value;
+    // p and dS of a half, piece by piece, beside the products from the first of its dP on (slot 0) to the end of the part
+    // behind that
+    auto soft = [&](auto half_c, auto slot_c) __attribute__((always_inline)) {
+      constexpr int h2 = decltype(half_c)::value, sl = decltype(slot_c)::value;
+      constexpr int EX = 16 / NKK;                               // exponentials per slot
+      constexpr int P0 = NKK > 4 ? NKK + 4 : NKK + 3;            // dS: from this slot on
+      constexpr int PN = (8 + 2 * NKK - P0 - 1) / (2 * NKK - P0);  // pairs per slot
       f32x16& s = st[h2];
-      if constexpr (pc == 3) asm volatile("" : "+v"(s));  // its last product is three behind
-      if constexpr (pc >= 3 && pc < 19) s[pc - 3] = fast_exp2(s[pc - 3]);
-      if constexpr (pc == 19) {
+      if constexpr (sl == 3) asm volatile("" : "+v"(s));  // its last product is three behind
+      if constexpr (sl >= 3 && sl < NKK + 3) {
+#pragma unroll
+        for (int e = EX * (sl - 3); e < EX * (sl - 2); ++e) s[e] = fast_exp2(s[e]);
+      }
+      if constexpr (sl == NKK + 3) {
         asm volatile("" : "+v"(dp[h2]));
         if (need_mask) {
           const int lo = a_i - n0 - 4 * g, hi = b_i - n0 - 4 * g;
@@ -1446,39 +1463,49 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
           asm volatile("" : "+v"(s));
         }
       }
-      if constexpr (pc >= 20 && pc < 28) {
-        constexpr int w = pc - 20;
-        ds[h2][w >> 2][w & 3] = pack_bf16x2(dp[h2][2 * w] * s[2 * w], dp[h2][2 * w + 1] * s[2 * w + 1]);
-        if constexpr ((w & 3) == 3) mfma32_operand(ds[h2][w >> 2]);
+      if constexpr (sl >= P0) {
+#pragma unroll
+        for (int w = PN * (sl - P0); w < PN * (sl - P0 + 1) && w < 8; ++w) {
+          ds[h2][w >> 2][w & 3] = pack_bf16x2(dp[h2][2 * w] * s[2 * w], dp[h2][2 * w + 1] * s[2 * w + 1]);
+          if ((w & 3) == 3) mfma32_operand(ds[h2][w >> 2]);
+        }
       }
     };
+    // the next tile has landed (of the loads behind it kStages - 2 tiles are still under way) and everybody's reads of
+    // this one are done
     auto next_tile = [&]() __attribute__((always_inline)) {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * kLoads) : "memory");
       __syncthreads();
-      const uint32_t d = SM::kBuf - 2 * buf;
+      const uint32_t d = buf + SM::kBuf < NS * SM::kBuf ? SM::kBuf : (uint32_t)-(NS - 1) * SM::kBuf;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) kr[j] += d;
+      for (int j = 0; j < NR; ++j) kr[j] += d;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { tr0[j] += d; tr1[j] += d; }
-      buf = SM::kBuf - buf;
+      for (int j = 0; j < NT; ++j) { tr0[j] += d; tr1[j] += d; }
+      buf += d;
       n0 = __builtin_amdgcn_readfirstlane(n0 + TB);
     };
-    // (past the last tile: this one's loads again, nobody reads them)
-    auto ahead = [&]() __attribute__((always_inline)) { return n0 + TB < blk_b ? n0 + TB : n0; };
+    // the tile whose loads go out beside this one's products, and where to: the buffer the last tile left
+    // (past the last one: this tile's again, nobody reads them)
+    auto ahead = [&]() __attribute__((always_inline)) { return n0 + (NS - 1) * TB < blk_b ? n0 + (NS - 1) * TB : n0; };
+    auto behind = [&]() __attribute__((always_inline)) { return buf ? buf - SM::kBuf : (NS - 1) * SM::kBuf; };
     auto skip_to = [&](int stop) __attribute__((always_inline)) {
 #pragma unroll 1
       while (n0 < stop) {
         const int n1 = ahead(), pl = place();
-        static_for<0, 16>([&](auto j) __attribute__((always_inline)) { issue(pl, n1, SM::kBuf - buf, j); });
+        static_for<0, kLoads>([&](auto j) __attribute__((always_inline)) { issue(pl, n1, behind(), j); });
         next_tile();
       }
     };
     __syncthreads();  // a previous pass may still be reading its buffers
     {
       const int pl = place();
-      static_for<0, 16>([&](auto j) __attribute__((always_inline)) { issue(pl, n0, 0, j); });
+      static_for<0, NS - 1>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int ti = decltype(tc)::value;
+        const int n = n0 + ti * TB < blk_b ? n0 + ti * TB : n0;
+        static_for<0, kLoads>([&](auto j) __attribute__((always_inline)) { issue(pl, n, ti * SM::kBuf, j); });
+      });
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * kLoads) : "memory");
     __syncthreads();
     skip_to(min(w_amin - TB + 1, blk_b));
     const int seen = min(w_bmax, blk_b);
@@ -1488,10 +1515,11 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
       do {
         need_mask = (n0 < w_amax) || (n0 + TB > w_bmin);
         const int n1 = ahead(), pl = place();
-        static_for<0, 96>([&](auto fc) __attribute__((always_inline)) {
-          constexpr int f = decltype(fc)::value, i = f & 15, part = f >> 4;
+        const uint32_t to = behind();
+        static_for<0, 6 * NKK>([&](auto fc) __attribute__((always_inline)) {
+          constexpr int f = decltype(fc)::value, i = f % NKK, part = f / NKK, kEnd = 6 * NKK, kSync = kEnd - RG / 2;
           using I = std::integral_constant<int, i>;
-          using I16 = std::integral_constant<int, i + 16>;
+          using I2 = std::integral_constant<int, i + NKK>;
           using H0 = std::integral_constant<int, 0>;
           using H1 = std::integral_constant<int, 1>;
           slots();
@@ -1502,19 +1530,19 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
             if constexpr (i == 0) mfma32_from(dp[part >> 1], fr[f % RG], dof[0][i], ndel[0]);
             else mfma32_onto(dp[part >> 1], fr[f % RG], dof[0][i]);
           } else {
-            mfma32_onto_v(acc[0][i & 7], fr[f % RG], as_bf16x8(ds[part - 4][i >> 3]));
+            mfma32_onto_v(acc[0][i % NDB], fr[f % RG], as_bf16x8(ds[part - 4][i / NDB]));
           }
           slots();
-          if constexpr (f + RG < 96) fread(std::integral_constant<int, f + RG>{});
+          if constexpr (f + RG < kEnd) fread(std::integral_constant<int, f + RG>{});
           if constexpr (part == 1) soft(H0{}, I{});
-          if constexpr (part == 2) soft(H0{}, I16{});
+          if constexpr (part == 2) soft(H0{}, I2{});
           if constexpr (part == 3) soft(H1{}, I{});
-          if constexpr (part == 4) soft(H1{}, I16{});
-          if constexpr (part < 2 && i % 2 == 0) issue(pl, n1, SM::kBuf - buf, std::integral_constant<int, part * 8 + i / 2>{});
-          if constexpr (f == 88) next_tile();
-          if constexpr (f >= 88) {
-            fread(std::integral_constant<int, 2 * (f - 88)>{});
-            fread(std::integral_constant<int, 2 * (f - 88) + 1>{});
+          if constexpr (part == 4) soft(H1{}, I2{});
+          if constexpr (f < 2 * kLoads && f % 2 == 0) issue(pl, n1, to, std::integral_constant<int, f / 2>{});
+          if constexpr (f == kSync) next_tile();
+          if constexpr (f >= kSync) {
+            fread(std::integral_constant<int, 2 * (f - kSync)>{});
+            fread(std::integral_constant<int, 2 * (f - kSync) + 1>{});
           }
         });
         slots();
@@ -1522,9 +1550,10 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
       mfma32_drain(acc[0]);
     }
     skip_to(blk_b);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (nothing may land in memory that is used for something else next)
   };
 
-  if constexpr (D > 128) {
+  if constexpr (SM::kWide) {
 #pragma unroll 1
     for (int c = 0; c < (p.a2 ? 2 : 1); ++c)  // (one copy of the code for both interval classes)
       wide_pass(c ? rb.a2[0] : rb.a1[0], c ? rb.b2[0] : rb.b1[0], c ? rb.w_a2min : rb.w_a1min, c ? rb.w_a2max : rb.w_a1max,

@@ -1,5 +1,5 @@
-"""Attention at head_dim 256 (``wide_pass`` of ``attn_fwd_kernel`` and ``attn_bwd_dq_kernel``: the products of a tile in one row
-with everything else spread beside them) against the explicit soft-max in float64 over the same rounded queries: odd row
+"""Attention at head_dim 256 (``wide_pass`` of ``attn_fwd_kernel`` and ``attn_bwd_dq_kernel``, the latter at 64 too: the products of
+a tile in one row with everything else spread beside them) against the explicit soft-max in float64 over the same rounded queries: odd row
 counts around the 32-key halves, 64-key tiles and 128-row workgroups, rows and whole tiles a wave sees nothing of, and
 scores whose maximum moves on in every half tile, in one jump, or never."""
 
@@ -28,25 +28,24 @@ def _reference(q, k, v, dense, scale, go):
     return out.transpose(1, 2).cpu(), dq.cpu(), bound.cpu()
 
 
-def _rows(t, hq, hkv, kind, steps=1):
+def _rows(t, hq, hkv, kind, d=256):
     g = torch.Generator().manual_seed(t + 7 * hq)
-    q, k, v = (torch.randn(1, h, n, 256, generator=g) for h, n in ((hq, t), (hkv, steps * t), (hkv, steps * t)))
+    q, k, v = (torch.randn(1, h, t, d, generator=g) for h in (hq, hkv, hkv))
     if kind != "flat":
         # a direction every query shares; the keys' share of it grows, falls, or jumps once: scores from 0 to about
         # +- 90 in steps the reference value has to follow (it is left alone up to a distance of 12 in the exponent of 2)
-        u = torch.randn(256, generator=g)
+        u = torch.randn(d, generator=g)
         u /= u.norm()
-        n = steps * t
-        ramp = {"rise": torch.linspace(0., 1., n), "fall": torch.linspace(1., 0., n),
-                "jump": (torch.arange(n) == 2 * n // 3).float()}[kind]
+        ramp = {"rise": torch.linspace(0., 1., t), "fall": torch.linspace(1., 0., t),
+                "jump": (torch.arange(t) == 2 * t // 3).float()}[kind]
         q += 8 * u
-        k += (ramp * 125)[None, None, :, None] * u
+        k += (ramp * 7.8 * d ** 0.5)[None, None, :, None] * u
     return tuple(x.bfloat16() for x in (q, k, v))
 
 
 def _check(fn, q, k, v, mask, dense):
-    scale = 256 ** -0.5
-    go = torch.randn(1, q.shape[2], q.shape[1], 256, generator=torch.Generator().manual_seed(1)).bfloat16()
+    scale = q.shape[3] ** -0.5
+    go = torch.randn(1, q.shape[2], q.shape[1], q.shape[3], generator=torch.Generator().manual_seed(1)).bfloat16()
     qg = q.cuda().requires_grad_(True)
     out = fn(qg, k.cuda(), v.cuda(), mask, scale)
     out.backward(go.cuda())
@@ -58,23 +57,25 @@ def _check(fn, q, k, v, mask, dense):
     assert torch.isfinite(qg.grad).all() and (off <= bound).all(), ((off - bound).max().item(), off.max().item())
 
 
+@pytest.mark.parametrize("d", [256, 64])
 @pytest.mark.parametrize("kind", ["flat", "rise", "fall", "jump"])
 @pytest.mark.parametrize("t,window,docs", [(1, None, 1), (31, None, 1), (33, None, 2), (64, None, 1), (97, 20, 1), (130, None, 3),
                                            (257, 40, 1), (333, None, 4), (1700, 100, 2), (1900, None, 1), (4977, None, 2)])
-def test_rows_and_reference_moves(t, window, docs, kind):
+def test_rows_and_reference_moves(t, window, docs, kind, d):
     from oracle import masks as OMK
     from speculators_amd import attention as A
 
     hq, hkv = (64, 2) if t > 4000 else (8, 2) if t > 1000 else (4, 1)  # (from 1.56e9 scores on V comes out of a transposed copy)
     doc = torch.arange(t) * docs // t
-    q, k, v = _rows(t, hq, hkv, kind)
+    q, k, v = _rows(t, hq, hkv, kind, d)
     mask = A.create_ttt_mask(doc.cuda(), t, window)
     _check(A.ttt_attention, q, k, v, mask, OMK.ttt_mask_dense(doc, t, 0, window))
 
 
+@pytest.mark.parametrize("d", [256, 64])
 @pytest.mark.parametrize("kind", ["flat", "rise"])
 @pytest.mark.parametrize("t,window", [(200, None), (777, 64)])
-def test_two_intervals_per_row(t, window, kind):
+def test_two_intervals_per_row(t, window, kind, d):
     """Anchored blocks: context keys and the block's own keys are two passes over one accumulator."""
     from oracle import masks as OMK
     from speculators_amd import attention as A
@@ -82,7 +83,7 @@ def test_two_intervals_per_row(t, window, kind):
     anchors = torch.arange(0, t - 1, 13)
     nq = 8 * len(anchors)
     doc = (torch.arange(t) > t // 3).long()
-    q, _, _ = _rows(nq, 4, 2, kind)
-    _, k, v = _rows(t + nq, 4, 2, kind)
+    q, _, _ = _rows(nq, 4, 2, kind, d)
+    _, k, v = _rows(t + nq, 4, 2, kind, d)
     mask = A.create_dflash_mask(doc.cuda(), t, anchors.cuda(), 8, window)
     _check(A.dflash_attention, q, k, v, mask, OMK.dflash_mask_dense(doc, t, anchors, 8, window))
