@@ -737,13 +737,10 @@ class _HeadLabelCE(torch.autograd.Function):
 
 # Whether the frozen-head cross-entropy takes its row statistics from the head product's epilogue
 # (spx_gemm_bf16_nt_stats, log-sum-exp only) instead of a streaming pass over the logits
-# (spx_label_ce_fwd).  Measured at the MTP head shape (32760 rows x 2048 -> 151936, 70 % live rows):
-# product + epilogue statistics + their reduction + one element per row 18.3 ms, product 17.3 ms +
-# streaming pass 1.3 ms = 18.6 ms back to back; inside the iteration the order is the other way by now, 196.1
-# against 194.4 ms.  (With the arg-max computed too and a reduction of one thread per row the epilogue form
-# LOST 1 ms per step: two compares per element more on every row, with the matrix pipe idle, cost what the
-# streaming pass costs.)
-HEAD_CE_EPILOGUE_STATS = True
+# (spx_label_ce_fwd).  The epilogue's exponentials hold the matrix pipe up for as long as the streaming pass takes
+# where live rows are 70 %: one iteration of the MTP head (three steps, 32760 rows x 2048 -> 151936) 186.3 ms with
+# the epilogue, 185.6 streaming; 2 x 4096 rows 38.6 and 38.2; 2000 rows, two steps 7.64 and 7.45; 600 rows 5.38 and 5.29.
+HEAD_CE_EPILOGUE_STATS = False
 
 
 def head_label_cross_entropy(x: torch.Tensor, weight: torch.Tensor, weight_t: torch.Tensor,
