@@ -243,8 +243,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(NormBwdSet one, NormBwd
 // thread j adds the slots j, j + 128, ..., then the 128 partial sums are combined through LDS
 // in a fixed order.  A latency-bound read of few megabytes by few workgroups: 1024 threads have
 // eight loads each to wait for at 1024 slots (256 threads had 32: 11.6 us at H = 4096, 3.5 us now).
-// A model's gains end in one launch after the backward: fourteen gains of three layers of width 2048 14 x 5 -> 18 us, and
-// their launches and casts off the host's path.
+// Gains whose gradients are ready together end in one launch: fourteen of three layers of width 2048 14 x 5 -> 18 us, and their
+// launches and casts off the host's path.
 constexpr int kSumSets = 16;
 struct SumSets {
   const float* part[kSumSets];

@@ -153,6 +153,8 @@ class DFlashDecoderLayer(nn.Module):
         if step is not None and x.dtype == x_normed.dtype == ctx.dtype == torch.bfloat16:
             step.take_slots(x.shape[1])
             att, post = self.self_attn, self.post_attention_layernorm
+            # (layer by layer: their gradients are ready with the layer's weights', not at the end of the backward)
+            self._stager.gains((att.q_norm, att.k_norm, post, next_norm))
             return LY.run_normed(step, x, x_normed, ctx, None, att.q_norm.gain, att.k_norm.gain, post.gain, next_norm.gain)
         a = self.self_attn(x_normed, ctx, q_pos, kv_pos, inv_freq, mask)
         post = self.post_attention_layernorm
@@ -195,7 +197,6 @@ class DFlashDraftModel(nn.Module):
         # lm_head and the loss as one autograd node while the head is frozen and the loss is a single
         # fused reduction (False: always two nodes)
         self.fuse_head_loss = True
-        self._norms = [m for m in self.modules() if isinstance(m, RMSNorm)]  # staged together (WeightStager.gains)
 
     @property
     def mask_token_id(self) -> int:
@@ -260,7 +261,6 @@ class DFlashDraftModel(nn.Module):
         t = hidden_states.shape[1]
         bs = self.block_size
         self._stager.begin()
-        self._stager.gains(self._norms)
         hidden_states = compute_input(hidden_states)
         verifier_last_hidden_states = compute_input(verifier_last_hidden_states)
         if position_ids is None:

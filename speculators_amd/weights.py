@@ -435,10 +435,12 @@ class WeightStager:
 
     def gains(self, norms):
         """Stages the gains of these norms (modules with ``weight``) through one node where they train: one launch casts
-        them (four at a time) and one sums their gradients, where each alone takes three launches."""
+        them (four at a time) and one sums their gradients, where each alone takes three launches.  The node runs when
+        the last of their uses has run its backward: norms that belong together by that."""
         if not torch.is_grad_enabled():
             return
-        ps = {id(n.weight): n.weight for n in norms if n.weight.requires_grad and n.weight.is_cuda}.values()
+        ps = {id(n.weight): n.weight for n in norms if n.weight.requires_grad and n.weight.is_cuda
+              and ("gain", id(n.weight), False) not in self._fwd}.values()
         autocast = _autocast_bf16()
         ps = [p for p in ps if p.dtype == torch.bfloat16 or (autocast and p.dtype == torch.float32)]
         if len(ps) > 1 and all(p.device == ps[0].device for p in ps):
