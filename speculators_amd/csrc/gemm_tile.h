@@ -67,6 +67,7 @@ struct Operand {
   static constexpr int kBytes = kR * kTK * 2;         // per slab
   static constexpr int kLoads = kBytes / 1024 / kWaves;  // 1 KB wave-loads per wave and slab
   static_assert(kBytes % (1024 * kWaves) == 0, "whole wave-loads");
+  static_assert(!SLOW || (kR & (kR - 1)) == 0, "whole rows per wave-load");
   u32x4 rsrc;
   int off[kLoads];
   int kchunk[SLOW ? 1 : 2];  // first contraction index of this lane's chunk inside the slab (even / odd row groups)

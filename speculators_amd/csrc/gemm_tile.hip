@@ -208,7 +208,15 @@ static int launch_reduce(const char* fname, const float* ws, void* c, int64_t ld
 // input gradients, 14 configurations each; 5 - 15 % rms).  On those products the choice is within 1.2 % of the best
 // candidate in the geometric mean and 1.33 x the 256 x 256 kernel alone (512 x 6144 -> 2048: 45.4 -> 23 us; 360 live
 // rows x 32000 -> 2048: 177 -> 62; 2000 x 4096 -> 4096: 71 -> 57; 4096-row products keep the large tile).
-enum Tile { kBig = 0, k128x128, k256x128, k64x128, k256x256 };
+// The tiles of 192 rows are for the row counts whose 256-row tiles fill the chip badly -- 2817 .. 3072 rows to 4096 columns
+// are 192 tiles of 256 x 256 and exactly 256 of 192 x 256 -- fitted to 99 products of 512 .. 5000 rows (3.5 - 6 % rms).
+// Where they are taken, 101 products of 700 .. 5000 rows run in 0.92 of the choice without them (geometric mean, both forms
+// alike; the worst 1.04, 700 x 2048 -> 16384): a b^T 1300 x 8192 -> 6144 184 -> 115 us, 1700 x 5120 -> 5120 115 -> 75,
+// 2900 x 4096 -> 3072 87 -> 63, 3001 x 14336 -> 4096 301 -> 283; a b 1300 x 14336 -> 4096 164 -> 144, 2300 x 4096 -> 4096
+// 90 -> 80, 3001 x 28672 -> 4096 604 -> 556, 5000 x 8192 -> 2048 170 -> 155.
+// (Tiles of 128 x 192 and 256 x 192 are the choice for too few further products, and the slow operand of the second form
+// takes whole powers of two only.)
+enum Tile { kBig = 0, k128x128, k256x128, k64x128, k192x256, kFifth /* NT: 192 x 192, NN: 256 x 256 */, k192x128 /* NN */ };
 struct Config {
   int tm, tn, per_cu;
   float s0, s1, b;
@@ -216,12 +224,16 @@ struct Config {
 constexpr Config kNT[] = {{256, 256, 1, 1.18f, 0.23f, 6.9f},   // kBig: gemm_bf16.hip, its last round cut (tail_plan)
                           {128, 128, 1, 0.35f, 0.14f, 4.1f},
                           {256, 128, 1, 0.52f, 0.25f, 5.3f},
-                          {64, 128, 2, 0.18f, 0.42f, 3.0f}};
+                          {64, 128, 2, 0.18f, 0.42f, 3.0f},
+                          {192, 256, 1, 1.04f, 0.14f, 8.5f},
+                          {192, 192, 1, 0.61f, 0.23f, 7.0f}};
 constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (no 4-wave kernel of this form)
                           {128, 128, 1, 0.43f, 0.125f, 0.6f},
                           {256, 128, 1, 0.59f, 0.22f, 3.9f},
                           {64, 128, 2, 0.25f, 0.48f, 0.f},
-                          {256, 256, 1, 1.13f, 0.33f, 4.0f}};
+                          {192, 256, 1, 1.04f, 0.14f, 7.2f},
+                          {256, 256, 1, 1.13f, 0.33f, 4.0f},
+                          {192, 128, 1, 0.50f, 0.14f, 5.5f}};
 // Weight gradients (contraction slow in both operands): the candidates beside the 256 x 256 kernel of gemm_bf16_tn.hip,
 // which keeps whole rounds of its tiles and is given up only for a predicted tenth.  Fitted the same way to 128 products
 // (results of 1 .. 768 large tiles, 256 .. 20000 rows, up to 12 parts; 6 - 13 % rms).  Over them the choice takes 0.52 of that
@@ -250,6 +262,9 @@ static float predict(const Config& c, int64_t tiles, int slabs) {
 
 static float reduce_us(int64_t elements) { return 4.1f + 1.03e-6f * (float)elements; }
 
+// (form 2: b a^T with the count of rows on the device.  No tiles of 192 rows there: the 256 x 256 kernel cuts its contraction
+// by the rows that count, which the host does not know -- 3001 rows x 32000 -> 4096, two thirds of them counting: 516 us
+// in parts, 661 on 192 x 256 tiles.)
 static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, bool can_split) {
   const int slabs = (int)((K + kTK - 1) / kTK);
   const bool nn = form == 1;
@@ -268,7 +283,7 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
     best.us = predict(c, tiles - cut, slabs);
     if (cut) best.us += predict(c, cut * tp, (slabs + tp - 1) / tp) + reduce_us(cut * tp * 65536);
   }
-  for (int t = 1; t < (nn ? 5 : 4); ++t) {
+  for (int t = 1; t < (nn ? 7 : form == 2 ? (int)k192x256 : 6); ++t) {
     const Config& c = table[t];
     const int64_t tiles = ((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
     const int64_t cap = (int64_t)kCus * c.per_cu;
@@ -337,9 +352,11 @@ static int launch_dense(const char* fname, int tile, const Params& p, hipStream_
     case k128x128: return launch<128, 128, 2, 4, 4, 2, false, BT, 0, false>(fname, p, 1, st);
     case k256x128: return launch<256, 128, 4, 2, 3, 2, false, BT, 0, false>(fname, p, 1, st);
     case k64x128: return launch<64, 128, 2, 2, 3, 2, false, BT, 0, false>(fname, p, 1, st);
+    case k192x256: return launch<192, 256, 2, 4, 2, 2, false, BT, 0, false>(fname, p, 1, st);
     default:
-      if constexpr (BT) return launch<256, 256, 2, 4, 2, 2, false, true, 0, false>(fname, p, 1, st);
-      return fail_arg(fname, "no such tile");
+      if constexpr (!BT) return launch<192, 192, 4, 2, 3, 2, false, false, 0, false>(fname, p, 1, st);
+      if (tile == k192x128) return launch<192, 128, 2, 4, 4, 2, false, BT, 0, false>(fname, p, 1, st);
+      return launch<256, 256, 2, 4, 2, 2, false, BT, 0, false>(fname, p, 1, st);
   }
 }
 
@@ -400,7 +417,7 @@ extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const vo
   SPX_REQ_FN(max_parts >= 1 && max_parts <= 8, "max_parts must be 1 .. 8");
   if (int rc = tile::dense_check(fname, form, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
   const bool vec = ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;  // (what the pass that adds the parts stores)
-  const tile::Choice ch = tile::choose(form, M, N, K, max_parts, can_split(N) && vec && workspace);
+  const tile::Choice ch = tile::choose(form == 0 && m_live ? 2 : form, M, N, K, max_parts, can_split(N) && vec && workspace);
   if (ch.tile == tile::kBig) {
     if (m_live) return spx_gemm_bf16_nt_rows(a, lda, b, ldb, c, ldc, M, N, K, m_live, stream);
     if (max_parts > 1 && workspace && workspace_bytes >= spx_gemm_tail_workspace_bytes())

@@ -140,7 +140,7 @@ def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = No
     if m_live is not None and (m_live.dtype != torch.int32 or m_live.numel() != 1 or m_live.device != a.device):
         raise ValueError("m_live must be a one-element int32 tensor on the operands' device")
     if k == b.shape[1] and k % 8 == 0 and a.stride(1) == 1 and b.stride(1) == 1 and a.dtype == b.dtype == torch.bfloat16:
-        big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
+        big, ws_numel, _ = _plan(0 if m_live is None else 2, m, n, k, TAIL_PARTS)
         if not big:
             return _auto(AUTO_NT, a, b, ws_numel, m_live)
     return gemm_nt(a, b, m_live=m_live, split=m_live is not None)
