@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void dflash_ranges_kernel(
 // Eight bf16 values times a scalar, rounded back to bf16 (round to nearest even).  The queries
 // enter every score product as bf16(q * scale * log2 e): the forward, the dQ kernel (both scale
 // their register fragments with this function) and the dK/dV and diagonal-key kernels (which
-// read the copy the backward's prologue writes with it) must see the SAME rounded values, or the
+// read the copy the dQ kernel writes with it) must see the SAME rounded values, or the
 // probabilities the backward recomputes would not match the forward's log-sum-exp.
 __device__ __forceinline__ u32x4 scale_bf16x8(u32x4 raw, float c) {
   u32x4 w;

@@ -194,8 +194,7 @@ class DFlashDraftModel(nn.Module):
             p.requires_grad_(False)
         self.uses_sliding_window_attn = bool(config.sliding_layers)
         self.uses_full_attn = config.num_hidden_layers > len(config.sliding_layers)
-        # lm_head and the loss as one autograd node while the head is frozen and the loss is a single
-        # fused reduction (False: always two nodes)
+        # lm_head and the loss as one autograd node while the head is frozen (False: always two nodes)
         self.fuse_head_loss = True
 
     @property

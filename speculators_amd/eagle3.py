@@ -290,8 +290,7 @@ class Eagle3DraftModel(nn.Module):
         self.embed_tokens.weight.requires_grad_(config.embed_requires_grad)
         self.uses_sliding_window_attn = bool(config.sliding_layers)
         self.uses_full_attn = config.num_hidden_layers > len(config.sliding_layers)
-        # lm_head and the loss as one autograd node while the head is frozen and the loss is a single
-        # fused reduction (False: always two nodes)
+        # lm_head and the loss as one autograd node while the head is frozen (False: always two nodes)
         self.fuse_head_loss = True
         # True: every forward leaves its per-step draft logits ([1, T, Vd], detached) in
         # ``last_logits`` (for parity checks; the reference returns no logits either)

@@ -1,6 +1,6 @@
 """A draft decoder layer -- one TTT step of it, or one pass -- as ONE autograd node.
 
-The layer (models/eagle3/model_definitions.py:14-110) is nine launches forward and thirteen backward; as
+The layer (models/eagle3/model_definitions.py:14-110) is nine launches forward and eleven backward; as
 eight nodes of their own they cost more host time (a node's forward and backward 20 us, and the views,
 slot look-ups and gradient checks between them) than the kernels take up to a thousand tokens: at 512
 tokens of the 1B shape a step of forward and backward was 0.61 ms of host time, 0.33 ms as one node.

@@ -200,7 +200,7 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
         loss_config = {"kl_div": (L.kl_div_loss, 1.0)}
     head = None
     if isinstance(logits, Head):
-        # one node for head + loss only when the whole loss is one fused reduction
+        # one node for head + loss: a loss of one streaming reduction in its own form, the others as weighted terms
         (name0, (fn0, _w0)), = list(loss_config.items())[:1]
         frozen = logits.x.requires_grad and not logits.weight.requires_grad and logits.weight_t is not None
         if frozen and (len(loss_config) > 1 or name0 not in ("kl_div", "ce")):
