@@ -663,7 +663,8 @@ int spx_gemm_bf16_nt(const void* a, int64_t lda, const void* b, int64_t ldb,
  * of that form's last round; 1: no contraction is ever cut.  m_live (device, may be NULL): the rows that count, as for
  * spx_gemm_bf16_nt_rows.  workspace: spx_gemm_auto_workspace_bytes() bytes, 16-byte aligned (may be NULL when that is
  * 0; a NULL workspace otherwise means no cut).  spx_gemm_auto_us: the predicted time in microseconds;
- * spx_gemm_auto_tile: 0 when the product runs on the 256 x 256 kernel of spx_gemm_bf16_nt.  These three (only) know a
+ * spx_gemm_auto_tile: 0 when the product runs on the 256 x 256 kernel of spx_gemm_bf16_nt, 5 in form 0 on tiles of
+ * 192 x 192.  These three (only) know a
  * form 2: form 0 with an m_live. */
 int64_t spx_gemm_auto_workspace_bytes(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts);
 float spx_gemm_auto_us(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts);

@@ -302,16 +302,23 @@ if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
     raise ValueError(f"SPX_DECODER_GEMM must be 'hipblaslt', 'spx' or 'mixed', got {DECODER_GEMM!r}")
 
 
+@functools.lru_cache(maxsize=4096)
+def _two_rounds_192(m: int, n: int, k: int, parts: int) -> bool:
+    return -(-m // 192) * -(-n // 192) <= 2 * _CUS and _lib.load().spx_gemm_auto_tile(0, m, n, k, parts) == 5
+
+
 def _own_forward(m: int, n: int, k: int) -> bool:
     """Whether the forward product of a decoder projection runs on this library's kernels in "mixed": where the
     smaller tiles fill the chip in one round (0.57 - 1.07 of hipBLASLt's time for the 1B, 8B and 70B shapes at 256 to
     8192 rows, 0.57 - 1.00 where the contraction is cut), and where the last round of the large tiles is cut along the
     contraction (``spx_gemm_bf16_nt_tail``; the merged q/k/v projection of the 8B shape: 291 us at 4096 rows, library
-    300).  Whole rounds of the large tiles mostly take 1.01 - 1.13 of the library's time.
+    300), and on at most two rounds of 192 x 192 tiles (1B q/k/v at 2900 - 3001 rows 0.83 of the library, 8B q/k/v at
+    1536 - 3001 0.88 - 0.97).  Whole rounds of the large tiles mostly take 1.01 - 1.13 of the library's time, of 192 x 256
+    tiles 0.94 - 1.07 (once 0.74, once 1.23).
     (All of them: profiles/decoder_forward_products.txt.)"""
     big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
     if not big:
-        return ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128
+        return ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128 or _two_rounds_192(m, n, k, TAIL_PARTS)
     tiles = -(-m // 256) * -(-n // 256)
     return TAIL_PARTS > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS
 

@@ -11,6 +11,14 @@ SHAPES = [  # (form, tile, M, N, K)
     (1, 4, 2903, 4088, 1032), (1, 4, 1537, 6152, 1032), (1, 6, 1300, 3080, 1032), (1, 6, 2689, 1544, 1032), (1, 6, 190, 10248, 4104)]
 
 
+def test_forward_projections_on_192_x_192_tiles():
+    from speculators_amd import gemm
+
+    # (rows, N, K): two rounds, one round, more than two rounds (library), 192 x 256 tiles (library)
+    for m, n, k, own in ((3001, 6144, 8192, True), (2900, 3072, 4096, True), (1300, 57344, 8192, False), (3001, 4096, 4096, False)):
+        assert gemm._own_forward(m, n, k) == own, (m, n, k)
+
+
 @pytest.mark.parametrize("form,tile,m,n,k", SHAPES)
 @pytest.mark.parametrize("pad", [0, 8, 3])
 @pytest.mark.parametrize("live", [None, 0, 1, 193, 5000])
