@@ -25,11 +25,12 @@ touches is *staged* once per forward:
     returns an equally empty marker for it so that the node is reached.  A use whose input
     is not in the buffer (nobody asked for the slot, or it was full) is added by a product of
     its own (accumulating in fp32);
-  * frozen weights (``lm_head``, ``verifier_lm_head``, ``embed_tokens``, ``verifier_norm``) are
+  * frozen weights (``lm_head``, ``verifier_lm_head``, ``embed_tokens``) are
     cast (and transposed where the backward needs it) once and kept until the parameter changes:
     the key is ``(data_ptr, _version, dtype)``; ``WeightStager.invalidate()`` drops every kept
     copy, and the models call it from ``train()`` / ``eval()`` and ``load_state_dict`` so that a
     write through ``param.data`` (which does not bump ``_version``) is picked up at those points.
+    Frozen norm gains are cast by every forward: a cast of a few KB is no reason to miss such a write.
 """
 
 from __future__ import annotations
@@ -429,7 +430,7 @@ class WeightStager:
             if plus_one:
                 hit = (1.0 + p.float()).to(torch.bfloat16)
             else:
-                hit = p if p.dtype == torch.bfloat16 else self.get(p).w  # (frozen: its copy is kept)
+                hit = p if p.dtype == torch.bfloat16 else p.to(torch.bfloat16)
             self._fwd["gain", id(p), plus_one] = hit
         return hit
 
