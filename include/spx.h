@@ -327,7 +327,8 @@ int spx_block_reduce(const float* loss, const int32_t* argmax_draft,
  * (from_anchor; losses/utils.py:17-48).  out [9 + 2 * block_size]: the two scalars of spx_block_reduce, then
  *   out[2] = *total_out = factor * out[0] (+ *total_in),  out[3], out[4] = matches, rows over the slots that count (all,
  *   or all but slot 0),  out[5] = sum of the running products of their accuracies,  out[6 .. 8] = 1,
- *   out[9 + s], out[9 + block_size + s] = matches, rows of slot s. */
+ *   out[9 + s], out[9 + block_size + s] = matches, rows of slot s.
+ * gamma may be any number, as there: negative, zero (weights of 0 and NaN), infinite. */
 int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target, const void* mask,
                     int mask_kind, const float* pos_weight, float gamma, int from_anchor, int64_t rows,
                     int32_t block_size, float factor, const float* total_in, float* total_out, float* out,

@@ -1293,7 +1293,8 @@ __global__ __launch_bounds__(NT) void row_tokens_kernel(const int32_t* __restric
 
 // What spx_block_total adds to the reduction of a block batch (scalars == nullptr: nothing).
 struct BlockTotal {
-  float gamma;            // > 0: the weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0; from_anchor: exp(-s / gamma)
+  int by_slot;            // the weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0; from_anchor: exp(-s / gamma)
+  float gamma;            // (any number: a negative one lets the weights grow)
   int from_anchor;
   float factor;           // the term's weight in the loss
   const float* total_in;  // loss so far (nullptr: none)
@@ -1309,7 +1310,7 @@ __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
   __shared__ float fl[kReduceThreads / 64];
   extern __shared__ int slots[];  // [2 * block_size], and a weight per slot behind them
   float* const decay = reinterpret_cast<float*>(slots + 2 * block_size);
-  const bool by_slot = bt.gamma > 0.f;
+  const bool by_slot = bt.by_slot;
   for (int i = threadIdx.x; i < 2 * block_size; i += kReduceThreads) slots[i] = 0;
   if (by_slot)
     for (int i = threadIdx.x; i < block_size; i += kReduceThreads)
@@ -1845,8 +1846,7 @@ extern "C" int spx_block_total(const float* loss, const int32_t* argmax_draft, c
                                int64_t rows, int32_t block_size, float factor, const float* total_in,
                                float* total_out, float* out, float* row_weight, void* stream) {
   SPX_REQUIRE(total_out && out && row_weight, "null buffer");
-  SPX_REQUIRE(pos_weight || gamma > 0.f, "a weight per row or a positive gamma");
-  const BlockTotal bt = {pos_weight ? 0.f : gamma, from_anchor, factor, total_in, total_out, out + 2};
+  const BlockTotal bt = {!pos_weight, gamma, from_anchor, factor, total_in, total_out, out + 2};
   return block_reduce(__func__, loss, argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
                       out + 9, out + 9 + block_size, row_weight, bt, stream);
 }
