@@ -1379,11 +1379,12 @@ __global__ __launch_bounds__(256) void dflash_inputs_kernel(
   const int64_t r = i - T;
   if (r >= n_q) return;
   const int j = (int)(r / block_size), s = (int)(r % block_size);
-  int64_t a = anchors[j];
+  int64_t a = anchors[j], row = a + s;
+  const bool inside = a >= -T && row < T;
+  if (row < 0) row += T;  // (counted from the end row by row: a block that begins in front of the end goes on at the start)
   if (a < 0) a += T;
-  const bool inside = a >= 0 && a + s < T;
   a = min(max(a, (int64_t)0), T - 1);
-  const int64_t row = min(a + s, T - 1);
+  row = min(max(row, (int64_t)0), T - 1);
   ids[r] = s == 0 ? input_ids[a] : mask_token;
   kv_pos[i] = positions[a] + s;
   target_row[r] = from_anchor ? row : row > 0 ? row - 1 : T - 1;

@@ -249,6 +249,23 @@ class DFlashDraftModel(nn.Module):
             aligned *= valid.to(dev, torch.float32).reshape(-1).repeat_interleave(bs)
         return out_ids.view(1, n_q), kv_pos[t:], kv_pos, idx, aligned
 
+    def _indexed_inputs(self, input_ids, position_ids, loss_mask, anchors, valid, t: int):
+        """``_inputs`` by plain indexing: ids and a loss mask of lengths of their own (each only has to reach as far as the
+        anchors and their blocks do), on another device, and what indexing refuses."""
+        bs = self.block_size
+        ids = torch.full((1, anchors.numel() * bs), self.mask_token_id, dtype=torch.long,
+                         device=self.embed_tokens.weight.device)
+        ids[:, ::bs] = input_ids[:, anchors]
+        block_pos = get_base_indices_for_anchored_blocks(position_ids[0, anchors], bs)
+        kv_pos = torch.cat([position_ids.reshape(-1), block_pos]).to(torch.int64).contiguous()
+        block_idx = get_base_indices_for_anchored_blocks(anchors, bs)
+        idx = block_idx if self.config.sample_from_anchor else (block_idx - 1) % t
+        aligned = loss_mask[:, block_idx]
+        aligned = aligned * valid.repeat_interleave(bs).unsqueeze(0).to(aligned.dtype)
+        if not self.config.sample_from_anchor:
+            aligned[:, ::bs] = 0
+        return ids, block_pos.to(torch.int64).contiguous(), kv_pos, idx, aligned
+
     def forward(self, hidden_states, input_ids, loss_mask, verifier_last_hidden_states,
                 document_ids, position_ids=None, loss_config: L.LossConfig | None = None,
                 gamma: float = 4.0, max_anchors: int = 512,
@@ -273,7 +290,11 @@ class DFlashDraftModel(nn.Module):
         sw_mask = (A.create_dflash_mask(doc, t, anchor_pos, bs, cfg.sliding_window,
                                         cfg.sliding_window_non_causal)
                    if self.uses_sliding_window_attn else None)
-        ids, q_pos, kv_pos, idx, aligned = self._inputs(input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t)
+        common = (input_ids.shape == position_ids.shape == loss_mask.shape == (1, t) and anchor_pos.dim() == 1
+                  and anchor_pos.dtype in (torch.int64, torch.int32) and anchor_valid.numel() == anchor_pos.numel()
+                  and input_ids.device == position_ids.device == loss_mask.device == device)
+        ids, q_pos, kv_pos, idx, aligned = (self._inputs if common else self._indexed_inputs)(
+            input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t)
         with torch.no_grad():
             noise = F.embedding(ids, self.embed_tokens.weight).to(hidden_states.dtype)
         ctx = self.hidden_norm(self._linear(hidden_states, self.fc.weight))
