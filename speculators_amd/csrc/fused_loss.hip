@@ -1370,7 +1370,8 @@ __global__ __launch_bounds__(256) void dflash_inputs_kernel(
     const int64_t* __restrict__ anchors, const uint8_t* __restrict__ valid, int n_q, int block_size, int64_t T,
     int64_t mask_token, const int64_t* __restrict__ input_ids, const int64_t* __restrict__ positions,
     const void* __restrict__ loss_mask, int mask_kind, int from_anchor, int64_t* __restrict__ ids,
-    int64_t* __restrict__ kv_pos, int64_t* __restrict__ target_row, float* __restrict__ aligned) {
+    int64_t* __restrict__ kv_pos, int64_t* __restrict__ target_row, float* __restrict__ aligned,
+    int32_t* __restrict__ outside) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < T) {
     kv_pos[i] = positions[i];
@@ -1381,6 +1382,7 @@ __global__ __launch_bounds__(256) void dflash_inputs_kernel(
   const int j = (int)(r / block_size), s = (int)(r % block_size);
   int64_t a = anchors[j], row = a + s;
   const bool inside = a >= -T && row < T;
+  if (!inside && outside) *outside = 1;
   if (row < 0) row += T;  // (counted from the end row by row: a block that begins in front of the end goes on at the start)
   if (a < 0) a += T;
   a = min(max(a, (int64_t)0), T - 1);
@@ -1855,7 +1857,7 @@ extern "C" int spx_block_total(const float* loss, const int32_t* argmax_draft, c
 extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
                                  int64_t T, int64_t mask_token, const int64_t* input_ids, const int64_t* positions,
                                  const void* loss_mask, int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos,
-                                 int64_t* target_row, float* aligned, void* stream) {
+                                 int64_t* target_row, float* aligned, int32_t* outside, void* stream) {
   SPX_REQUIRE(T > 0 && T < (1ll << 30) && n_anchors >= 0 && block_size > 0 && n_anchors * block_size < (1ll << 30),
               "sizes out of range");
   SPX_REQUIRE(input_ids && positions && loss_mask && kv_pos && kind_ok(mask_kind), "null buffer or unknown mask kind");
@@ -1863,6 +1865,6 @@ extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, i
   const int64_t n_q = n_anchors * block_size;
   hipLaunchKernelGGL(dflash_inputs_kernel, dim3((unsigned)((T + n_q + 255) / 256)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), anchors, valid, (int)n_q, block_size, T, mask_token,
-                     input_ids, positions, loss_mask, mask_kind, from_anchor, ids, kv_pos, target_row, aligned);
+                     input_ids, positions, loss_mask, mask_kind, from_anchor, ids, kv_pos, target_row, aligned, outside);
   return check_launch(__func__);
 }

@@ -83,6 +83,40 @@ def select_anchors(loss_mask: torch.Tensor, num_anchors: int, block_size: int):
     return anchors, ok
 
 
+def _check_reach(anchors: torch.Tensor, *spans):
+    """IndexError where a block leaves what it indexes; ``spans`` are pairs of a length and how many rows from an anchor on are
+    read of it (rows below 0 count from the end).  Waits for the anchors."""
+    if anchors.dtype not in (torch.int64, torch.int32) or anchors.numel() == 0:
+        return
+    if anchors.is_cuda and torch.cuda.is_current_stream_capturing():
+        return
+    first, last = (int(x) for x in torch.aminmax(anchors.cpu()))
+    for length, rows in spans:
+        if first < -length or last + rows > length:
+            raise IndexError(f"anchors {first} .. {last}: {rows} rows from each on do not fit {length}")
+
+
+class _Outside:
+    """Where the launch that makes a step's inputs says that an anchor's block leaves the sequence: a word of pinned host
+    memory, read at the end of the forward, when that launch has long run or the whole forward is still queued behind it.
+    (Three 1B-shape layers over 1777 rows: 2.79 -> 2.82 ms a step; 2.9 with a copy of the anchors in the place of the word.)"""
+
+    def __init__(self, device):
+        self.word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.done, self.device = torch.cuda.Event(), device
+
+    def launched(self):
+        self.done.record(torch.cuda.current_stream(self.device))
+
+    def settle(self):
+        self.done.synchronize()
+        if self.word.item():
+            raise IndexError("an anchor's block leaves the sequence")
+
+    def __del__(self):
+        self.done.synchronize()  # (a forward that ended early: the word is not given back under the launch)
+
+
 @LY.passed_by
 class DFlashAttention(nn.Module):
     """q from the mask tokens; k/v from ``cat([context, mask tokens])``; per-head q/k
@@ -224,7 +258,7 @@ class DFlashDraftModel(nn.Module):
         """``x @ weight.T`` on the MFMA kernel of this library (fc, lm_head, verifier head)."""
         return gemm.linear_staged(x, self._stager.get(weight), hip=True)
 
-    def _inputs(self, input_ids, position_ids, loss_mask, anchors, valid, t: int):
+    def _inputs(self, input_ids, position_ids, loss_mask, anchors, valid, t: int, outside: _Outside | None = None):
         """``(ids [1, n_q], q_pos [n_q], kv_pos [t + n_q], target rows [n_q], aligned loss mask [1, n_q])`` of the blocks
         that start at ``anchors`` (models/dflash/core.py:264-271,330-439)."""
         dev, bs, cfg = input_ids.device, self.block_size, self.config
@@ -244,7 +278,9 @@ class DFlashDraftModel(nn.Module):
         aligned = torch.empty(1, n_q, device=dev, dtype=torch.float32)
         _lib.call("spx_dflash_inputs", row(anchors.to(dev)), row(valid.to(dev), torch.bool), anchors.numel(), bs, t,
                   int(self.mask_token_id), ids, pos, mask, _lib.kind_code(mask), int(cfg.sample_from_anchor), out_ids,
-                  kv_pos, idx, aligned, _lib.stream_ptr(dev))
+                  kv_pos, idx, aligned, None if outside is None else outside.word.data_ptr(), _lib.stream_ptr(dev))
+        if outside is not None:
+            outside.launched()
         if valid.dtype != torch.bool:  # (weights instead of flags)
             aligned *= valid.to(dev, torch.float32).reshape(-1).repeat_interleave(bs)
         return out_ids.view(1, n_q), kv_pos[t:], kv_pos, idx, aligned
@@ -253,6 +289,8 @@ class DFlashDraftModel(nn.Module):
         """``_inputs`` by plain indexing: ids and a loss mask of lengths of their own (each only has to reach as far as the
         anchors and their blocks do), on another device, and what indexing refuses."""
         bs = self.block_size
+        spans = [(input_ids.shape[-1], 1), (position_ids.shape[-1], 1), (loss_mask.shape[-1], bs)]
+        _check_reach(anchors, *spans, *([(t, bs)] if self.config.sample_from_anchor else []))
         ids = torch.full((1, anchors.numel() * bs), self.mask_token_id, dtype=torch.long,
                          device=self.embed_tokens.weight.device)
         ids[:, ::bs] = input_ids[:, anchors]
@@ -271,7 +309,8 @@ class DFlashDraftModel(nn.Module):
                 gamma: float = 4.0, max_anchors: int = 512,
                 per_position_loss_weight: str = "fixed-exp-decay", dpace_alpha: float = 0.5,
                 anchors=None, **_kwargs):
-        """``anchors=(positions, valid)`` overrides the random anchor selection."""
+        """``anchors=(positions, valid)`` overrides the random anchor selection; one whose block leaves the sequence is an
+        IndexError."""
         cfg = self.config
         device = hidden_states.device
         t = hidden_states.shape[1]
@@ -281,7 +320,8 @@ class DFlashDraftModel(nn.Module):
         verifier_last_hidden_states = compute_input(verifier_last_hidden_states)
         if position_ids is None:
             position_ids = torch.arange(t, dtype=torch.long, device=device).unsqueeze(0)
-        if anchors is None:
+        given = anchors is not None
+        if not given:
             anchors = select_anchors(loss_mask, max_anchors, bs)
         anchor_pos, anchor_valid = anchors
         doc = document_ids.reshape(-1).to(device)
@@ -293,8 +333,16 @@ class DFlashDraftModel(nn.Module):
         common = (input_ids.shape == position_ids.shape == loss_mask.shape == (1, t) and anchor_pos.dim() == 1
                   and anchor_pos.dtype in (torch.int64, torch.int32) and anchor_valid.numel() == anchor_pos.numel()
                   and input_ids.device == position_ids.device == loss_mask.device == device)
-        ids, q_pos, kv_pos, idx, aligned = (self._inputs if common else self._indexed_inputs)(
-            input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t)
+        # (the model's own anchors fit by themselves, but for a sequence shorter than a block; in a captured graph nothing can be
+        # waited for, and the loss is NaN)
+        outside = None
+        if common:
+            if (given or bs > t) and not torch.cuda.is_current_stream_capturing():
+                outside = _Outside(device)
+            inputs = self._inputs(input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t, outside)
+        else:
+            inputs = self._indexed_inputs(input_ids, position_ids, loss_mask, anchor_pos, anchor_valid, t)
+        ids, q_pos, kv_pos, idx, aligned = inputs
         with torch.no_grad():
             noise = F.embedding(ids, self.embed_tokens.weight).to(hidden_states.dtype)
         ctx = self.hidden_norm(self._linear(hidden_states, self.fc.weight))
@@ -320,6 +368,8 @@ class DFlashDraftModel(nn.Module):
             logits, targets, aligned, bs, gamma=gamma, loss_config=loss_config,
             per_position_loss_weight=per_position_loss_weight, dpace_alpha=dpace_alpha,
             sample_from_anchor=cfg.sample_from_anchor)
+        if outside is not None:
+            outside.settle()
         return None, loss, metrics
 
     @staticmethod

@@ -1,5 +1,5 @@
 """Calls of the anchored-block model and its metrics off the common form: inputs of other lengths and shapes, anchors counted
-from the end, and decay rates that are not positive."""
+from the end, decay rates that are not positive, and anchors whose block leaves the sequence."""
 
 import pytest
 import torch
@@ -81,6 +81,17 @@ def test_two_rows_of_ids_are_refused():
     b = _batch()
     with pytest.raises((RuntimeError, ValueError)):
         _step(_model(), dict(b, input_ids=b["input_ids"].view(2, T // 2)), [1, 17])
+
+
+@pytest.mark.parametrize("anchors", [[1, T - BS + 1], [T + 3], [-T - 1, 4]])
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+@pytest.mark.parametrize("extra", [0, 7])
+def test_a_block_that_leaves_the_sequence_is_refused(anchors, where, extra):
+    model, batch = _model(), _batch(extra, 0)
+    a = torch.tensor(anchors, device=where)
+    with pytest.raises(IndexError):
+        model(**batch, anchors=(a, torch.ones(len(anchors), dtype=torch.bool, device=where)))
+    _step(model, batch, [1, T - BS])  # (the last one that fits; nothing is left behind)
 
 
 @pytest.mark.parametrize("gamma", [-3.0, float("inf"), 0.0, float("nan")])
