@@ -121,7 +121,7 @@ int spx_vocab_loss_step_fwd(int op, const void* logits, int64_t ld_logits,
  *                                softmax(logits[r]) - onehot(argmax targets[r])     (ce)
  * i.e. the gradient for a row weight of ONE: what follows is linear in the rows, so the weight
  * the reduction behind the loss gives row r is applied to the result of the input-gradient
- * product (spx_unpack_rows_graded).  Rows mapped to -1 get no gradient row; with
+ * product (spx_gemm_bf16_rows_graded).  Rows mapped to -1 get no gradient row; with
  * reuse_target_stats their target row is not read and their loss and lse_draft are written as 0
  * (a masked row's loss enters no sum), their arg-max outputs and chain update are as for any
  * row. */
@@ -299,9 +299,12 @@ int spx_ttt_step_terms(int32_t terms, const float* term_weights, const float* lo
                        float* out, float* row_weight, void* stream);
 
 /* spx_pack_row_map for a row mask of any element kind (live: not zero); zero3 (int32[3], may be NULL) is
- * cleared: the counts of the loss pass that follows. */
+ * cleared: the counts of the loss pass that follows.  spx_mask_row_lists: also row_of[s] = the live row in slot s
+ * (int32 [rows], slots past the count are not written). */
 int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
                      int32_t* zero3, void* stream);
+int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
+                       int32_t* row_of, int32_t* zero3, void* stream);
 
 /* Draft tokens: out[i] = known[i] for i < n (int32 arg-maxes of a loss pass, widened), out[n + j] = the first
  * index of the maximum of row j < tail of rows[tail, vocab] (bf16 / f32, row stride ld). */
@@ -734,6 +737,17 @@ int spx_gemm_bf16_nt_rows_split(const void* a, int64_t lda, const void* b, int64
                                 const int32_t* m_live, int32_t max_parts, void* workspace,
                                 int64_t workspace_bytes, void* stream);
 
+/* The product of packed rows that were made for unit weights (spx_vocab_loss_step_fwd_grad,
+ * spx_vocab_loss_terms_fwd_grad): row m of c is row row[m] of the whole and is multiplied by
+ * row_weight[row[m]] * (*scale * factor) in fp32, before its one rounding.  Tiles and parts as spx_gemm_bf16_auto chooses
+ * them in form 2 (max_parts: as there; workspace: spx_gemm_auto_workspace_bytes(2, ..) bytes, NULL: no cut), on the
+ * 256 x 256 kernel as spx_gemm_bf16_nt_rows_split with split_parts where the workspace holds them (split_parts * M * N
+ * floats), else as spx_gemm_bf16_nt_rows.  m_live, row, row_weight and scale are device memory. */
+int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
+                              int64_t N, int64_t K, const int32_t* m_live, const int32_t* row, const float* row_weight,
+                              const float* scale, float factor, int32_t max_parts, int32_t split_parts, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+
 /* The two ends of a packed-rows product (spx_*_bwd_packed -> spx_gemm_bf16_nt_rows).
  * spx_pack_row_map: row_map[r] = number of live rows before r if row r is live
  * (row_grad[r] != 0 and, when labels is not NULL, labels[r] != ignore_index), else -1;
@@ -751,11 +765,6 @@ int spx_unpack_rows(const void* packed, int64_t ld_packed, const int32_t* row_ma
 int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, const int32_t* row_map,
                            const float* row_scale, int64_t rows, int64_t total_rows,
                            int64_t cols, void* out, int64_t ld_out, void* stream);
-
-/* The same with row_scale[r] * (*scale * factor); scale: one f32 on the device (NULL: 1 and no factor). */
-int spx_unpack_rows_graded(const void* packed, int64_t ld_packed, const int32_t* row_map,
-                           const float* row_scale, const float* scale, float factor, int64_t rows,
-                           int64_t total_rows, int64_t cols, void* out, int64_t ld_out, void* stream);
 
 /* c[M, N] (+)= a[T, M]^T * b[T, N], bf16 inputs, fp32 accumulation, bf16 output:
  * the weight-gradient product of the backward of torch.nn.Linear (dW = dY^T X)

@@ -47,6 +47,7 @@ SIGNATURES["spx_block_total"] = [_P, _P, _P, _P, _I, _P, _F, _I, _I64, _I32, _F,
 SIGNATURES["spx_dflash_inputs"] = [_P, _P, _I64, _I32, _I64, _I64, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_ttt_step_terms"] = [_I32, _P, _P, _P, _I, _I64, _F, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_map"] = [_P, _I, _I64, _P, _P, _P, _P]
+SIGNATURES["spx_mask_row_lists"] = [_P, _I, _I64, _P, _P, _P, _P, _P]
 SIGNATURES["spx_row_tokens"] = [_P, _I64, _P, _I64, _I64, _I64, _I, _P, _P]
 SIGNATURES["spx_span_attn_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _F, _P, _P,
                                    _P, _I64, _P]
@@ -93,7 +94,6 @@ SIGNATURES["spx_pack_batch"] = [_P, _I, _I64, _I64, _I64, _P, _P, _I, _P, _P, _P
 SIGNATURES["spx_gemm_bf16_nt"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]
 SIGNATURES["spx_pack_row_map"] = [_P, _P, _I64, _I64, _P, _P, _P]
 SIGNATURES["spx_unpack_rows"] = [_P, _I64, _P, _I64, _I64, _I64, _P, _I64, _P]
-SIGNATURES["spx_unpack_rows_graded"] = [_P, _I64, _P, _P, _P, _F, _I64, _I64, _I64, _P, _I64, _P]
 SIGNATURES["spx_unpack_rows_scaled"] = [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I64, _P]
 SIGNATURES["spx_vocab_loss_step_fwd_grad"] = [_I, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _I,
                                               _P, _I, _P, _I, _P, _P, _P, _I64, _P]
@@ -105,6 +105,8 @@ SIGNATURES["spx_gemm_bf16_nt_stats"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64
 SIGNATURES["spx_gemm_stats_workspace_bytes"] = [_I64, _I64]
 SIGNATURES["spx_gemm_bf16_nt_rows"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _P]
 SIGNATURES["spx_gemm_bf16_nt_rows_split"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P]
+SIGNATURES["spx_gemm_bf16_rows_graded"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _F, _I32, _I32, _P,
+                                           _I64, _P]
 SIGNATURES["spx_gemm_bf16_tn"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _P]
 SIGNATURES["spx_gemm_bf16_tn_auto"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P]
 SIGNATURES["spx_gemm_tn_parts"] = [_I64, _I64, _I64]

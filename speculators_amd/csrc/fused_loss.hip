@@ -452,8 +452,8 @@ __global__ __launch_bounds__(NT) void loss_fwd_kernel(
 // bf16), reduces it to the row statistics exactly like loss_fwd_kernel, and, for a row that row_map
 // sends to a slot >= 0, goes over its registers a second time and writes
 //   grad[slot, :] = softmax(x) - softmax(y)   (kl)      softmax(x) - onehot(argmax y)   (ce)
-// -- the gradient for a row weight of ONE; the caller applies the weight the reduction behind the loss
-// gives the row to the input-gradient product's result (which is linear in it).  Rows mapped to -1 get
+// -- the gradient for a row weight of ONE; the input-gradient product, which is linear in it, applies the weight the reduction
+// behind the loss gives the row to its fp32 sums, before their one rounding (spx_gemm_bf16_rows_graded).  Rows mapped to -1 get
 // no gradient row, and with the target statistics handed in (KNOWN) their target row is not read at
 // all, no soft-max of their draft row is formed and their loss is written as zero: a masked row's loss enters
 // no sum.  (Their arg-max outputs and their part of the acceptance chain are those of any row.)
@@ -1249,9 +1249,10 @@ __global__ __launch_bounds__(kReduceThreads) void ttt_step_terms_kernel(
 // The rows a mask leaves, in order, and three zeroed counters for the loss pass behind it.
 __global__ __launch_bounds__(1024) void mask_row_map_kernel(const void* __restrict__ mask, int mask_kind, int rows,
                                                             int32_t* __restrict__ row_map,
-                                                            int32_t* __restrict__ count, int32_t* __restrict__ zero3) {
+                                                            int32_t* __restrict__ count,
+                                                            int32_t* __restrict__ row_of, int32_t* __restrict__ zero3) {
   if (zero3 && threadIdx.x < 3) zero3[threadIdx.x] = 0;
-  pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, rows, row_map, count);
+  pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, rows, row_map, count, row_of);
 }
 
 // Draft tokens (int64): the known arg-maxes of the first n rows widened, the arg-max (first index of the
@@ -1787,13 +1788,18 @@ extern "C" int spx_ttt_step_terms(int32_t terms, const float* term_weights, cons
   return check_launch(__func__);
 }
 
-extern "C" int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
-                                int32_t* zero3, void* stream) {
+extern "C" int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
+                                  int32_t* row_of, int32_t* zero3, void* stream) {
   SPX_REQUIRE(rows > 0 && rows < (1ll << 31), "rows out of range");
   SPX_REQUIRE(mask && row_map && count && kind_ok(mask_kind), "null buffer or unknown mask element kind");
   hipLaunchKernelGGL(mask_row_map_kernel, dim3(1), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), mask,
-                     mask_kind, (int)rows, row_map, count, zero3);
+                     mask_kind, (int)rows, row_map, count, row_of, zero3);
   return check_launch(__func__);
+}
+
+extern "C" int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
+                                int32_t* zero3, void* stream) {
+  return spx_mask_row_lists(mask, mask_kind, rows, row_map, count, nullptr, zero3, stream);
 }
 
 extern "C" int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail,

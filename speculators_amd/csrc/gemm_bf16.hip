@@ -130,14 +130,16 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
   tile_n = m_long ? sh : l;
 }
 
-template <bool kImm, int kStats = 0>
+// kGrade: the rows are multiplied by their factors (RowGrade) on the way to their rounding.
+template <bool kImm, int kStats = 0, bool kGrade = false>
 __global__ __launch_bounds__(kGemmThreads, SPX_GEMM_MINW)
 __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf16_nt_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
     uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K, int tiles_m, int tiles_n,
     const int32_t* __restrict__ m_live, const int32_t* __restrict__ tile_tab,
     const int32_t* __restrict__ group_off, int64_t b_group_stride, float* __restrict__ part_ws,
-    int max_parts, int cus, float* __restrict__ stat_ws = nullptr, int tail_mode = 0) {
+    int max_parts, int cus, float* __restrict__ stat_ws = nullptr, int tail_mode = 0,
+    RowGrade grade = {}) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int M_host = M;
   // the row count may live on the device (rows packed to the front by the producer of A): the tile
@@ -400,12 +402,24 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   float* const st_lds = reinterpret_cast<float*>(smem);  // [wave][3][128]
   if constexpr (kStats != 0) __syncthreads();
   const bool edge_n = n0 + kTN > N;
+  float by[kMI];
+  if constexpr (kGrade) {
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+      const int m = m0 + wm + i * 16 + r16;
+      by[i] = m < M ? grade.at(m) : 0.f;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < kMI; ++i) {
     const int m = m0 + wm + i * 16 + r16;
     uint32_t pk[kNI][2];
 #pragma unroll
     for (int j = 0; j < kNI; ++j) {
+      if constexpr (kGrade) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][i][r] *= by[i];
+      }
       pk[j][0] = pack_bf16x2(acc[j][i][0], acc[j][i][1]);
       pk[j][1] = pack_bf16x2(acc[j][i][2], acc[j][i][3]);
     }
@@ -600,7 +614,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
                                                                  uint16_t* __restrict__ C, int64_t ldc, int M_host,
                                                                  int N, int K, int tiles_n,
                                                                  const int32_t* __restrict__ m_live, int max_parts,
-                                                                 int cus) {
+                                                                 int cus, RowGrade grade) {
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
   const int parts = choose_k_parts(((M + kTM - 1) / kTM) * tiles_n, max_parts, cus, (K + kTK - 1) / kTK);
   if (parts <= 1) return;
@@ -614,6 +628,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
     lo[0] += a[0]; lo[1] += a[1]; lo[2] += a[2]; lo[3] += a[3];
     hi[0] += b[0]; hi[1] += b[1]; hi[2] += b[2]; hi[3] += b[3];
+  }
+  if (grade.row) {
+    const float by = grade.at(m);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { lo[r] *= by; hi[r] *= by; }
   }
   u32x4 v;
   v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
@@ -646,7 +665,8 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
                         int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live, void* stream,
                         const int32_t* tile_tab = nullptr, const int32_t* group_off = nullptr,
                         int64_t b_group_stride = 0, int64_t groups = 0, float* part_ws = nullptr,
-                        int max_parts = 1, float* stat_ws = nullptr, int stats_mode = 0, int tail_mode = 0) {
+                        int max_parts = 1, float* stat_ws = nullptr, int stats_mode = 0, int tail_mode = 0,
+                        const RowGrade& grade = RowGrade{}) {
   SPX_REQ_FN(M > 0 && N > 0 && K > 0, "M, N, K must be positive");
   SPX_REQ_FN(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "dimension too large");
   SPX_REQ_FN(a && b && (c || stat_ws), "null buffer");
@@ -657,16 +677,18 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
              "256 rows of an operand must span less than 2 GiB (32-bit offsets inside a tile)");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool imm = lda >= kTK && ldb >= kTK;
-  static std::atomic<uint64_t> lds_set[8];  // per kernel instantiation, one bit per device
-  const int which = (imm ? 1 : 0) + 2 * (stat_ws ? stats_mode : 0);
-  const void* const fns[8] = {reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 0>),
+  static std::atomic<uint64_t> lds_set[10];  // per kernel instantiation, one bit per device
+  const int which = (imm ? 1 : 0) + 2 * (stat_ws ? stats_mode : grade.row ? 4 : 0);
+  const void* const fns[10] = {reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 0>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 0>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 1>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 1>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 2>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 2>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 3>),
-                              reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 3>)};
+                              reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 3>),
+                              reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 0, true>),
+                              reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 0, true>)};
   if (int rc = ensure_dynamic_lds(fns[which], kGemmSmem, lds_set[which], fname)) return rc;
   // grouped: every group may end in a partly filled tile row
   const int64_t tiles_m64 = (M + kTM - 1) / kTM + (tile_tab ? groups : 0);
@@ -683,11 +705,11 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
     n_grid = (int64_t)tiles_m * tiles_n + (int64_t)(tiles_m * tiles_n - tail_first) * (tail_parts - 1);
   }
   const dim3 grid((unsigned)n_grid), block(kGemmThreads);
-#define SPX_GEMM_LAUNCH(IMM, STATS)                                                                              \
-  hipLaunchKernelGGL((gemm_bf16_nt_kernel<IMM, STATS>), grid, block, kGemmSmem, st,                              \
+#define SPX_GEMM_LAUNCH(IMM, ...)                                                                                \
+  hipLaunchKernelGGL((gemm_bf16_nt_kernel<IMM, __VA_ARGS__>), grid, block, kGemmSmem, st,                        \
                      reinterpret_cast<const uint16_t*>(a), lda, reinterpret_cast<const uint16_t*>(b), ldb,       \
                      reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_m, tiles_n, m_live,      \
-                     tile_tab, group_off, b_group_stride, part_ws, max_parts, cus, stat_ws, tail_mode)
+                     tile_tab, group_off, b_group_stride, part_ws, max_parts, cus, stat_ws, tail_mode, grade)
   switch (which) {
     case 0: SPX_GEMM_LAUNCH(false, 0); break;
     case 1: SPX_GEMM_LAUNCH(true, 0); break;
@@ -696,7 +718,9 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
     case 4: SPX_GEMM_LAUNCH(false, 2); break;
     case 5: SPX_GEMM_LAUNCH(true, 2); break;
     case 6: SPX_GEMM_LAUNCH(false, 3); break;
-    default: SPX_GEMM_LAUNCH(true, 3); break;
+    case 7: SPX_GEMM_LAUNCH(true, 3); break;
+    case 8: SPX_GEMM_LAUNCH(false, 0, true); break;
+    default: SPX_GEMM_LAUNCH(true, 0, true); break;
   }
 #undef SPX_GEMM_LAUNCH
   if (int rc = check_launch(fname)) return rc;
@@ -713,7 +737,7 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
   if (part_ws) {
     const int64_t items = M * (N / 8);
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, part_ws,
-                       reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_n, m_live, max_parts, cus);
+                       reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_n, m_live, max_parts, cus, grade);
     return check_launch(fname);
   }
   return 0;
@@ -852,5 +876,12 @@ extern "C" int spx_gemm_bf16_nt_rows(const void* a, int64_t lda, const void* b, 
     return SPX_ERR_ARG;
   }
   return gemm_nt_impl(__func__, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream);
+}
+
+int spx::nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+                        int64_t M, int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws,
+                        int max_parts, void* stream) {
+  return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream, nullptr, nullptr, 0, 0, part_ws,
+                      part_ws ? max_parts : 1, nullptr, 0, 0, grade);
 }
 #undef SPX_REQ_FN

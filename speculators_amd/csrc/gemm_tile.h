@@ -17,6 +17,7 @@
 // 3.2 TB/s as 64-byte pieces, 3.3 in whole lines, 3.6 past the caches and 4.6 with both.
 #pragma once
 
+#include "gemm_tile_api.h"
 #include "spx_common.h"
 
 namespace spx {
@@ -155,10 +156,12 @@ struct Params {
   const int32_t* group_off;     // grouped: group boundaries
   const int32_t* m_live;        // how many leading rows of A count (device; null: all M)
   int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)
+  RowGrade grade;               // GRADE: what the rows are multiplied by
 };
 
-// OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C.  STREAM: non-temporal stores (OUT 0 and 2)
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM>
+// OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C.  STREAM: non-temporal stores (OUT 0 and 2).  GRADE: rows
+// multiplied by their factors on the way to their rounding (OUT 0; of a product in parts the pass that adds them does it)
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE>
 __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p) {
   constexpr int kWaves = WM * WN, kMI = TM / WM / 16, kNI = TN / WN / 16;
   using OA = Operand<TM, kWaves, AT>;
@@ -406,6 +409,15 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
       }
     }
   } else {
+    if constexpr (GRADE) {
+#pragma unroll
+      for (int i = 0; i < kMI; ++i) {
+        const int m = m0 + wm + i * 16 + r16;
+        const float by = m < M ? p.grade.at(m) : 0.f;
+#pragma unroll
+        for (int j = 0; j < kNI; ++j) acc[j][i] *= by;
+      }
+    }
     uint16_t* const Cb = reinterpret_cast<uint16_t*>(C);
     const bool fast = (p.ldc % 8 == 0) && ((reinterpret_cast<uintptr_t>(Cb) & 15) == 0);
     // odd groups of 16 lanes of block j <-> even groups of block j + 1: 8 consecutive columns per lane

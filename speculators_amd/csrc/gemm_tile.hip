@@ -58,13 +58,13 @@ __global__ __launch_bounds__(256) void group_tiles_kernel(const int32_t* __restr
 
 constexpr int kCus = 256;
 
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM>
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE = false>
 static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
   constexpr int kSmem = (TM + TN) * kTK * 2 * STAGES;
   static std::atomic<uint64_t> lds_set;
-  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM>;
+  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmem, lds_set, fname)) return rc;
-  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM>),
+  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE>),
                      dim3((unsigned)(p.tiles_m * p.tiles_n * p.parts), (unsigned)groups_y), dim3(64 * WM * WN), kSmem,
                      st, p);
   return check_launch(fname);
@@ -157,11 +157,11 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
 
 // ------------------------------------------------------------------------------------------ plain products
 // C[m, n .. n + 7] = the sum of the parts of a product whose contraction was cut, in their order, fp32, one rounding.
-// OUT as in gemm_tile_kernel.
+// OUT as in gemm_tile_kernel; grade (OUT 0): what the rows of the sum are multiplied by.
 template <int OUT>
 __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ ws, void* __restrict__ C,
                                                            int64_t ldc, int M_host, int N, int parts,
-                                                           const int32_t* __restrict__ m_live) {
+                                                           const int32_t* __restrict__ m_live, RowGrade grade) {
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
   const int n8 = N / 8;
   const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -172,6 +172,11 @@ __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restri
     const float* src = ws + ((int64_t)p * M_host + m) * N + n;
     lo += *reinterpret_cast<const f32x4*>(src);
     hi += *reinterpret_cast<const f32x4*>(src + 4);
+  }
+  if (OUT == 0 && grade.row) {
+    const float by = grade.at(m);
+    lo *= by;
+    hi *= by;
   }
   if constexpr (OUT >= 2) {
     f32x4* const cp = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + (int64_t)m * ldc + n);
@@ -194,10 +199,10 @@ __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restri
 
 template <int OUT>
 static int launch_reduce(const char* fname, const float* ws, void* c, int64_t ldc, int64_t M, int64_t N, int parts,
-                         const int32_t* m_live, hipStream_t st) {
+                         const int32_t* m_live, hipStream_t st, const RowGrade& grade = RowGrade{}) {
   const int64_t items = M * (N / 8);
   hipLaunchKernelGGL(parts_reduce_kernel<OUT>, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, ws, c, ldc, (int)M,
-                     (int)N, parts, m_live);
+                     (int)N, parts, m_live, grade);
   return check_launch(fname);
 }
 
@@ -360,6 +365,15 @@ static int launch_dense(const char* fname, int tile, const Params& p, hipStream_
   }
 }
 
+// (the tiles of form 2)
+static int launch_graded(const char* fname, int tile, const Params& p, hipStream_t st) {
+  switch (tile) {
+    case k128x128: return launch<128, 128, 2, 4, 4, 2, false, false, 0, false, true>(fname, p, 1, st);
+    case k256x128: return launch<256, 128, 4, 2, 3, 2, false, false, 0, false, true>(fname, p, 1, st);
+    default: return launch<64, 128, 2, 2, 3, 2, false, false, 0, false, true>(fname, p, 1, st);
+  }
+}
+
 }  // namespace tile
 }  // namespace spx
 
@@ -444,6 +458,44 @@ extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const vo
     return rc;
   if (ch.parts == 1) return SPX_OK;
   return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st);
+}
+
+extern "C" int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+                                         int64_t M, int64_t N, int64_t K, const int32_t* m_live, const int32_t* row,
+                                         const float* row_weight, const float* scale, float factor, int32_t max_parts,
+                                         int32_t split_parts, void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* fname = __func__;
+  SPX_REQ_FN(max_parts >= 1 && max_parts <= 8 && split_parts >= 1 && split_parts <= 8, "parts must be 1 .. 8");
+  SPX_REQ_FN(m_live && row && row_weight && scale, "null row count, rows, weights or scale");
+  SPX_REQ_FN(!workspace || ((uintptr_t)workspace) % 16 == 0, "unaligned workspace");
+  if (int rc = tile::dense_check(fname, 0, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
+  const RowGrade grade = {row, row_weight, scale, factor};
+  const bool vec = ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;  // (what the pass that adds the parts stores)
+  const tile::Choice ch = tile::choose(2, M, N, K, max_parts, can_split(N) && vec && workspace);
+  const int64_t part = M * N * (int64_t)sizeof(float);
+  if (ch.tile == tile::kBig) {
+    const bool cut = split_parts > 1 && can_split(N) && vec && workspace && workspace_bytes >= split_parts * part;
+    return nt_rows_graded(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, grade,
+                          cut ? reinterpret_cast<float*>(workspace) : nullptr, split_parts, stream);
+  }
+  SPX_REQ_FN(ch.parts == 1 || workspace_bytes >= ch.parts * part, "workspace too small");
+  const tile::Config& cfg = tile::kNT[ch.tile];
+  tile::Params p{};
+  p.A = reinterpret_cast<const uint16_t*>(a);
+  p.B = reinterpret_cast<const uint16_t*>(b);
+  p.C = c;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.M = (int)M; p.N = (int)N; p.K = (int)K;
+  const int64_t tiles_m = (M + cfg.tm - 1) / cfg.tm, tiles_n = (N + cfg.tn - 1) / cfg.tn;
+  SPX_REQ_FN(tiles_m * tiles_n * ch.parts < (1ll << 31), "too many tiles");
+  p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n; p.parts = ch.parts;
+  p.part_ws = reinterpret_cast<float*>(workspace);
+  p.m_live = m_live;
+  p.grade = grade;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (int rc = tile::launch_graded(fname, ch.tile, p, st)) return rc;
+  if (ch.parts == 1) return SPX_OK;
+  return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st, grade);
 }
 
 // ------------------------------------------------------------------------------------------ weight gradients

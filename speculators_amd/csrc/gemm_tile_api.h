@@ -1,9 +1,26 @@
 // Entry points of gemm_tile.hip for the other GEMM sources (arguments as in the C entry points that call them).
 #pragma once
 
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace spx {
+
+// What the rows of a packed product are multiplied by before their one rounding: row m of the result is row row[m] of the
+// whole, with a weight of its own and a scalar on the device (row == nullptr: nothing).
+struct RowGrade {
+  const int32_t* row;
+  const float* weight;
+  const float* scale;
+  float factor;
+  __device__ __forceinline__ float at(int m) const { return weight[row[m]] * (*scale * factor); }
+};
+
+// spx_gemm_bf16_nt_rows (part_ws == nullptr) or spx_gemm_bf16_nt_rows_split with graded rows (gemm_bf16.hip)
+int nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
+                   int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws, int max_parts,
+                   void* stream);
+
 namespace tile {
 
 int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t b_group_stride,

@@ -346,7 +346,7 @@ PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // One TTT step's loss over bf16 logits in one read of the rows, with its masked mean: (op, logits, targets or None, known
 // lse_t, known argmax_t or None, mask, its kind, prev or None, its kind, acceptance counts or None (made and cleared here),
 // loss so far or None, step weight, term factor, scalars [8] or None: no mean) -> (total, row losses, argmax_draft,
-// argmax_target, lse_target, packed logits gradient, row map, live rows, row weights)
+// argmax_target, lse_target, packed logits gradient, row map, live rows, row weights, rows by slot)
 PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Args x("loss_step", args, n, 14);
@@ -363,17 +363,17 @@ PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool known = known_lse.defined();
   void* const st = stream_of(logits);
   const auto i32 = logits.options().dtype(at::kInt), f32 = logits.options().dtype(at::kFloat);
-  const Tensor map = at::empty({rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({5 * rows}, f32),
+  const Tensor map = at::empty({2 * rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({5 * rows}, f32),
                packed = at::empty({rows, vocab}, logits.options()), total = at::empty({}, f32);
-  int32_t* const row_map = map.mutable_data_ptr<int32_t>();
+  int32_t* const row_map = map.mutable_data_ptr<int32_t>();  // the map, the count, the rows by slot
   int32_t* const am = arg.mutable_data_ptr<int32_t>();
   int32_t* const counts = given.defined() ? given.mutable_data_ptr<int32_t>() : am + 2 * rows;
   float* const s = floats(stats);  // loss, lse_draft, lse_target, extra, row weights
   float* const lse_t = known ? known_lse.mutable_data_ptr<float>() : s + 2 * rows;
   int32_t* const am_t = known ? known_arg.mutable_data_ptr<int32_t>() : am + rows;
-  check(spx_mask_row_map(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows,
-                         given.defined() ? nullptr : counts, st),
-        "spx_mask_row_map");
+  check(spx_mask_row_lists(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows, row_map + rows + 1,
+                           given.defined() ? nullptr : counts, st),
+        "spx_mask_row_lists");
   check(spx_vocab_loss_step_fwd_grad(op, in(logits), logits.stride(0), y.defined() ? in(y) : nullptr,
                                      y.defined() ? y.stride(0) : 0, rows, vocab, s, s + rows, lse_t, s + 3 * rows, am, am_t,
                                      known, mask.const_data_ptr(), mask_kind,
@@ -388,7 +388,7 @@ PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return tuple_of(released, {total, stats.narrow(0, 0, rows), arg.narrow(0, 0, rows),
                              known ? known_arg : arg.narrow(0, rows, rows),
                              known ? known_lse : stats.narrow(0, 2 * rows, rows), packed, map.narrow(0, 0, rows),
-                             map.narrow(0, rows, 1), stats.narrow(0, 4 * rows, rows)});
+                             map.narrow(0, rows, 1), stats.narrow(0, 4 * rows, rows), map.narrow(0, rows + 1, rows)});
   END_HANDLE_TH_ERRORS
 }
 
@@ -413,7 +413,7 @@ PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
   bool known = known_lse.defined();
   void* const st = stream_of(logits);
   const auto i32 = logits.options().dtype(at::kInt), f32 = logits.options().dtype(at::kFloat);
-  const Tensor map = at::empty({rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({9 * rows}, f32),
+  const Tensor map = at::empty({2 * rows + 1}, i32), arg = at::empty({2 * rows + 3}, i32), stats = at::empty({9 * rows}, f32),
                packed = at::empty({rows, vocab}, logits.options()), total = at::empty({}, f32);
   int32_t* const row_map = map.mutable_data_ptr<int32_t>();
   int32_t* const am = arg.mutable_data_ptr<int32_t>();
@@ -421,7 +421,8 @@ PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
   float* const s = floats(stats);  // lse_draft, lse_target, row weights, one more, up to five terms' losses
   float* const lse_t = known ? known_lse.mutable_data_ptr<float>() : s + rows;
   int32_t* const am_t = known ? known_arg.mutable_data_ptr<int32_t>() : am + rows;
-  check(spx_mask_row_map(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows, counts, st), "spx_mask_row_map");
+  check(spx_mask_row_lists(mask.const_data_ptr(), mask_kind, rows, row_map, row_map + rows, row_map + rows + 1, counts, st),
+        "spx_mask_row_lists");
   Tensor gathered;
   if (d2t.defined()) {
     gathered = at::empty({rows, vocab}, logits.options());
@@ -445,7 +446,7 @@ PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool given = known_lse.defined();
   return tuple_of(released, {total, arg.narrow(0, 0, rows), given ? known_arg : arg.narrow(0, rows, rows),
                              given ? known_lse : stats.narrow(0, rows, rows), packed, map.narrow(0, 0, rows),
-                             map.narrow(0, rows, 1), stats.narrow(0, 2 * rows, rows), y});
+                             map.narrow(0, rows, 1), stats.narrow(0, 2 * rows, rows), map.narrow(0, rows + 1, rows), y});
   END_HANDLE_TH_ERRORS
 }
 

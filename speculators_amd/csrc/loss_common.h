@@ -106,11 +106,11 @@ __device__ __forceinline__ float mask_value(const void* p, int kind, int64_t i) 
   }
 }
 
-// row_map[r] = number of live rows before r if live(r), else -1; *count = number of live rows.  One workgroup
-// of 1024 threads, rows in order.
+// row_map[r] = number of live rows before r if live(r), else -1; *count = number of live rows; row_of (may be null) = the live
+// rows.  One workgroup of 1024 threads, rows in order.
 template <typename Live>
 __device__ __forceinline__ void pack_row_map(Live live_at, int rows, int32_t* __restrict__ row_map,
-                                             int32_t* __restrict__ count) {
+                                             int32_t* __restrict__ count, int32_t* __restrict__ row_of = nullptr) {
   __shared__ int wave_tot[16];
   __shared__ int base_s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -126,6 +126,7 @@ __device__ __forceinline__ void pack_row_map(Live live_at, int rows, int32_t* __
     int off = base_s;
     for (int w = 0; w < wave; ++w) off += wave_tot[w];
     if (r < rows) row_map[r] = live ? off + before : -1;
+    if (live && row_of) row_of[off + before] = r;
     __syncthreads();
     if (tid == 0) {
       int t = 0;

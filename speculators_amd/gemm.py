@@ -146,6 +146,29 @@ def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = No
     return gemm_nt(a, b, m_live=m_live, split=m_live is not None)
 
 
+def rows_graded(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor, row_of: torch.Tensor, row_weight: torch.Tensor,
+                scale: torch.Tensor, factor: float) -> torch.Tensor:
+    """``matmul_nt(a, b, m_live)`` with row ``m`` multiplied by ``row_weight[row_of[m]] * (scale * factor)`` in fp32, before its
+    one rounding (``spx_gemm_bf16_rows_graded``)."""
+    m, k = a.shape
+    n = b.shape[0]
+    if k != b.shape[1] or m_live.dtype != torch.int32 or row_of.dtype != torch.int32 or row_of.numel() < m:
+        raise ValueError(f"a {tuple(a.shape)}, b {tuple(b.shape)}, int32 row count and rows")
+    if row_weight.dtype != torch.float32 or scale.dtype != torch.float32 or not row_weight.is_contiguous():
+        raise ValueError("row weights and scale are contiguous fp32")
+    if b.stride(1) != 1:
+        b = b.contiguous()
+    big, ws_numel, _ = _plan(2, m, n, k, TAIL_PARTS)
+    if big:  # (as gemm_nt(split=True))
+        few_tiles = -(-m // 256) * -(-n // 256) <= 2 * _CUS
+        ws_numel = SPLIT_PARTS * m * n if SPLIT_PARTS > 1 and few_tiles and n % 8 == 0 and k >= 64 * 16 * 2 else 0
+    ws = _split_workspace(a.device, ws_numel) if ws_numel else None
+    out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
+    _lib.call("spx_gemm_bf16_rows_graded", a, a.stride(0), b, b.stride(0), out, n, m, n, k, m_live, row_of, row_weight, scale,
+              factor, TAIL_PARTS, SPLIT_PARTS, ws, ws.numel() * 4 if ws_numel else 0, _lib.stream_ptr(a.device))
+    return out
+
+
 def _nn_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether ``a[M, K] @ b[K, N]`` meets the alignment rules of the NN kernels."""
     k, n = b.shape

@@ -235,7 +235,8 @@ def _one_pass_ok(op, x, y, step) -> bool:
 
 def _loss_step(op, x, y, known, step, mean=None, total_in=None):
     """The row pass that also writes the unit-weight logits gradient of the unmasked rows, packed to the front, and
-    the masked mean behind it.  Returns ``(total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight)``."""
+    the masked mean behind it.  Returns ``(total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight, row_of)``
+    (``row_of``: the live rows in their order)."""
     rows = x.shape[0]
     lse_t = am_t = None
     if known is not None:
@@ -250,7 +251,7 @@ def _loss_step(op, x, y, known, step, mean=None, total_in=None):
 
 def _loss_forward_with_grad(op, x, y, known, step):
     """``_loss_step`` without the mean: ``(loss, lse_t, am_d, am_t, packed, row_map, count)``."""
-    _, loss, am_d, am_t, lse_t, packed, row_map, count, _ = _loss_step(op, x, y, known, step)
+    _, loss, am_d, am_t, lse_t, packed, row_map, count, *_ = _loss_step(op, x, y, known, step)
     return loss, lse_t, am_d, am_t, packed, row_map, count
 
 
@@ -364,15 +365,12 @@ class BlockTerm:
 
 
 def _unit_rows_backward(saved, g32, factor: float, total_rows: int):
-    """dx of the frozen head from the unit-weight logits gradient of the live rows that the row pass left behind."""
-    from .gemm import matmul_nt
+    """dx of the frozen head from the unit-weight logits gradient of the live rows that the row pass left behind: the row
+    weights go onto the product's fp32 sums, so that dx is rounded once."""
+    from .gemm import rows_graded
 
-    packed, row_map, count, weight_t, row_weight = saved
-    dx_packed = matmul_nt(packed, weight_t, m_live=count)
-    dx = torch.empty(total_rows, dx_packed.shape[1], device=packed.device, dtype=packed.dtype)
-    _lib.call("spx_unpack_rows_graded", dx_packed, dx_packed.stride(0), row_map, row_weight, g32, factor,
-              row_map.numel(), total_rows, dx.shape[1], dx, dx.stride(0), _lib.stream_ptr(dx.device))
-    return dx
+    packed, row_map, count, weight_t, row_weight, row_of = saved
+    return _unpack_rows(rows_graded(packed, weight_t, count, row_of, row_weight, g32, factor), row_map, total_rows)
 
 
 class _HeadStepLoss(torch.autograd.Function):
@@ -381,7 +379,7 @@ class _HeadStepLoss(torch.autograd.Function):
 
     Where it can (``_one_pass_ok``) the forward reads the rows once for everything: loss, statistics, acceptance
     chain and the unit-weight logits gradient of the unmasked rows, packed to the front; the backward is then the
-    input-gradient product of the head and the unpacking of its rows, which applies the row weights."""
+    input-gradient product of the head, which applies the row weights, and the unpacking of its rows."""
 
     @staticmethod
     def forward(ctx, x2, total_in, weight, weight_t, targets, op, known, n_rows, step, mean):
@@ -394,11 +392,11 @@ class _HeadStepLoss(torch.autograd.Function):
         ctx.one_pass = ((known is not None or targets is not None) and _one_pass_ok(op, xs, targets, step)
                         and (not blocks or xs.shape[1] >= TERMS_MIN_VOCAB))
         if ctx.one_pass:
-            total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight = _loss_step(
+            total, loss, am_d, am_t, lse_t, packed, row_map, count, row_weight, row_of = _loss_step(
                 op, xs, targets, known, step, None if blocks else mean, total_in)
             if blocks:
                 total, row_weight = mean.reduce(loss, am_d, am_t, None, total_in)
-            ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
+            ctx.save_for_backward(packed, row_map, count, weight_t, row_weight, row_of)
         else:
             if blocks:
                 step = None
@@ -476,11 +474,11 @@ class _HeadTermsLoss(torch.autograd.Function):
         for op, w in terms:
             weights[op] = w
         lse_t, am_t = (None, None) if known is None else (known[0].reshape(-1), known[1].reshape(-1))
-        total, am_d, am_t, lse_t, packed, row_map, count, row_weight, rows = _lib.native().loss_terms(
+        total, am_d, am_t, lse_t, packed, row_map, count, row_weight, row_of, rows = _lib.native().loss_terms(
             sum(1 << op for op, _ in terms), *weights, logits[:n_rows], targets, d2t, lse_t, am_t, step.mask,
             _lib.kind_code(step.mask), step.prev, _lib.kind_code(step.prev) if step.prev is not None else 0, total_in,
             step_weight, out)
-        ctx.save_for_backward(packed, row_map, count, weight_t, row_weight)
+        ctx.save_for_backward(packed, row_map, count, weight_t, row_weight, row_of)
         if d2t is not None:
             step.gathered = rows
         ctx.mark_non_differentiable(am_d, am_t, lse_t, logits)
