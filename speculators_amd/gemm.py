@@ -326,24 +326,38 @@ if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
 
 
 @functools.lru_cache(maxsize=4096)
-def _two_rounds_192(m: int, n: int, k: int, parts: int) -> bool:
-    return -(-m // 192) * -(-n // 192) <= 2 * _CUS and _lib.load().spx_gemm_auto_tile(0, m, n, k, parts) == 5
+def _on_192_rows(m: int, n: int, k: int, parts: int) -> bool:
+    """The part of ``_own_forward`` for products that the tiles of 192 rows took from whole rounds of the large ones."""
+    tile = _lib.load().spx_gemm_auto_tile(0, m, n, k, parts)
+    if tile == 5 and -(-m // 192) * -(-n // 192) <= 2 * _CUS:
+        return True
+    return tile in (4, 5) and m <= 1024 and k <= 3072
 
 
 def _own_forward(m: int, n: int, k: int) -> bool:
-    """Whether the forward product of a decoder projection runs on this library's kernels in "mixed": where the
-    smaller tiles fill the chip in one round (0.57 - 1.07 of hipBLASLt's time for the 1B, 8B and 70B shapes at 256 to
-    8192 rows, 0.57 - 1.00 where the contraction is cut), and where the last round of the large tiles is cut along the
-    contraction (``spx_gemm_bf16_nt_tail``; the merged q/k/v projection of the 8B shape: 291 us at 4096 rows, library
-    300), and on at most two rounds of 192 x 192 tiles (1B q/k/v at 2900 - 3001 rows 0.83 of the library, 8B q/k/v at
-    1536 - 3001 0.88 - 0.97).  Whole rounds of the large tiles mostly take 1.01 - 1.13 of the library's time, of 192 x 256
-    tiles 0.94 - 1.07 (once 0.74, once 1.23).
-    (All of them: profiles/decoder_forward_products.txt.)"""
-    big, ws_numel, _ = _plan(0, m, n, k, TAIL_PARTS)
+    """Whether the forward product of a decoder projection runs on this library's kernels in "mixed" (ratios: own time to
+    hipBLASLt's).
+
+    Chosen without the tiles of 192 rows: where smaller tiles fill the chip in one round (0.54 - 1.04 for 70 products of the
+    1B, 8B and 70B shapes at 256 to 4096 rows, three 1.11 - 1.20), and where the last round of the large tiles is cut along
+    the contraction (``spx_gemm_bf16_nt_tail``; 0.67 - 1.16 for 15, the merged q/k/v projection of the 8B shape at 4096 rows
+    0.96).  What these choose may then run on tiles of 192 rows.
+
+    Of the rest, whole rounds of the large tiles (mostly 1.01 - 1.13), what the tiles of 192 rows took: at most two rounds
+    of 192 x 192 (29 products of 140 to 8199 rows 0.51 - 1.02, 0.81 in the geometric mean; 1B q/k/v at 2700 - 3072 rows 0.84 -
+    0.91, 8B q/k/v at 1350 - 1536 0.92), and up to 1024 rows where the contraction is short: K to 3072 0.57 - 1.05 over 30
+    products (0.83), from 4096 on 0.80 - 1.33 over 41 (1.06; 8B gate/up at 260 - 960 rows 0.99 - 1.11, 70B q/k/v at 777 - 1024
+    1.24 - 1.33, 70B gate/up 1.02 - 1.21).
+    (profiles/decoder_forward_products.txt.)"""
+    big, ws_numel, _ = _plan(2, m, n, k, TAIL_PARTS)  # (the choice without them is that of a device row count)
     if not big:
-        return ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128 or _two_rounds_192(m, n, k, TAIL_PARTS)
-    tiles = -(-m // 256) * -(-n // 256)
-    return TAIL_PARTS > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS
+        if ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128:
+            return True
+    else:
+        tiles = -(-m // 256) * -(-n // 256)
+        if TAIL_PARTS > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS:
+            return True
+    return _on_192_rows(m, n, k, TAIL_PARTS)
 
 
 def _project(x2: torch.Tensor, staged) -> torch.Tensor:

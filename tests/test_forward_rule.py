@@ -1,0 +1,27 @@
+"""Which decoder projections run on this library's kernels forward ("mixed"): a rule of sizes alone, no GPU needed."""
+
+import random
+
+import pytest
+
+from speculators_amd import _lib, gemm
+
+
+@pytest.mark.parametrize("rows,n,k,own", [
+    # up to 1024 rows on tiles of 192 rows: 70B q/k/v and gate/up and 8B gate/up stay with the library, short contractions do not
+    (777, 10240, 16384, False), (1024, 10240, 16384, False), (1024, 10240, 8192, False), (160, 57344, 8192, False),
+    (384, 57344, 8192, False), (260, 28672, 4096, False), (384, 28672, 4096, False), (888, 28672, 4096, False),
+    (600, 16384, 2048, True), (768, 16384, 2048, True),
+    # two rounds of 192 x 192, a contraction in parts, a cut last round, smaller tiles
+    (3001, 6144, 8192, True), (1300, 4096, 14336, True), (4096, 6144, 8192, True), (512, 6144, 8192, True), (1024, 2048, 2048, True)])
+def test_measured_products(rows, n, k, own):
+    assert gemm._own_forward(rows, n, k) == own
+
+
+def test_nothing_that_ran_here_without_the_tall_tiles_goes_to_the_library():
+    rnd = random.Random(1)
+    for _ in range(4000):
+        m, n, k = rnd.randint(8, 5000), 8 * rnd.randint(16, 4096), 8 * rnd.randint(64, 2048)
+        tile = _lib.load().spx_gemm_auto_tile(2, m, n, k, gemm.TAIL_PARTS)  # the choice without tiles of 192 rows
+        if tile and m <= 1024:
+            assert gemm._own_forward(m, n, k), (m, n, k)
