@@ -688,7 +688,8 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
   // like this (62 % at 1.7 GHz: at the power limit); 600 rows 32.0 and 23.0.  The soft-max inside its own tile (two quarters
   // without it, two with all of it) 1946; a ring of eight operands instead of sixteen 1 % more; V^T out of rows of the whole
   // length, 64 bytes per load and row, in the place of blocks of 32 keys 12 % more.
-  auto wide_pass = [&](int a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
+  // (auto: head sizes that do not call it get no body of it, whose fragments their arrays have no room for)
+  auto wide_pass = [&](auto a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
     static_assert(NSB == 1, "one 32-row block per wave");
     if (blk_b <= blk_a) return;
     constexpr int RG = 16;
@@ -1386,7 +1387,8 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_d
   // 512 rows 15.7 and 14.7, 4096 125 and 114, 8192 under a window of 2048 209 and 196.  At head_dim 128 this needs more
   // registers than two waves of a SIMD have, and with one wave a call of more than one workgroup per compute unit loses:
   // 4096 rows of 32 heads 227 and 233, 8192 of 64 1370 and 1424 (1024 of 32: 32.2 and 27.8).
-  auto wide_pass = [&](int a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
+  // (auto: head sizes that do not call it get no body of it, whose fragments their arrays have no room for)
+  auto wide_pass = [&](auto a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
     static_assert(NSB == 1, "one 32-row block per wave");
     if (blk_b <= blk_a) return;
     constexpr int RG = D > 64 ? 16 : 8, NS = SM::kStages;

@@ -1271,7 +1271,8 @@ __global__ __launch_bounds__(NT) void row_tokens_kernel(const int32_t* __restric
   const T* row = rows + (int64_t)blockIdx.x * ld;
   float best = -INFINITY;
   int at = 0x7fffffff;
-#pragma unroll(NT > 256 ? 4 : 1)
+  constexpr int kAhead = NT > 256 ? 4 : 1;
+#pragma unroll kAhead
   for (int64_t base = (int64_t)threadIdx.x * 8; base < vocab; base += NT * 8) {
     float x[8];
     load8<T, VEC>(row, base, vocab, x);

@@ -15,6 +15,14 @@ CSRC = os.path.join(ROOT, "speculators_amd", "csrc")
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("source", sorted(f for f in os.listdir(CSRC) if f.endswith(".hip")))
+def test_sources_compile_without_warnings(source):
+    """An index past the end of a register array, for one, is a warning and nothing else."""
+    subprocess.run(["hipcc", "-std=c++17", "--offload-arch=gfx950", "-fsyntax-only", "-Werror", "-Wno-unused-command-line-argument",
+                    os.path.join(CSRC, source)], check=True, capture_output=True)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_hand_issued_loads_are_not_read_before_their_wait(tmp_path):
     out = tmp_path / "fused_loss.s"
     subprocess.run(["hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature",
