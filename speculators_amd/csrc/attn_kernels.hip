@@ -301,6 +301,7 @@ __device__ __forceinline__ void mfma32_onto_v(f32x16& d, bf16x8 a, bf16x8 b) {  
 #endif
 // a product's operand is complete: not to be formed any later, and two issue slots from here to the product
 __device__ __forceinline__ void mfma32_operand(u32x4& x) { asm volatile("s_nop 1" : "+v"(x)); }
+__device__ __forceinline__ void mfma32_operand(f32x16& x) { asm volatile("s_nop 1" : "+v"(x)); }
 // every product under way has arrived
 template <int N>
 __device__ __forceinline__ void mfma32_drain(f32x16 (&d)[N]) {
@@ -835,8 +836,10 @@ __global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_
           for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[0][db][r] *= alpha;
-          mfma32_drain(st);
-          mfma32_drain(acc[0]);
+          // (a wait that does not name the registers leaves the compiler free to scale the last of them behind it)
+          mfma32_operand(nref[0]);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) mfma32_operand(acc[0][db]);
         }
         rs = 0.f;
       } else if constexpr (pc >= 7 && pc < 23) {

@@ -1,7 +1,9 @@
-"""A property of the compiled code that no numerical test pins reliably: in the pipelined gather
+"""Properties of the compiled code that no numerical test pins reliably.  In the pipelined gather
 kernel the registers written by the hand-issued table loads must not be read by any instruction
 before the ``s_waitcnt`` that releases them (a read before it returns whatever the register held,
-sometimes the right value).  The check compiles the source to gfx950 assembly and walks it."""
+sometimes the right value).  In the attention kernels whose matrix products are inline assembly, which
+the compiler takes for any other statement, the issue slots that such a product needs before and behind
+it must be there.  The checks compile the source to gfx950 assembly and walk it."""
 
 import os
 import re
@@ -22,14 +24,106 @@ def test_sources_compile_without_warnings(source):
                     os.path.join(CSRC, source)], check=True, capture_output=True)
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-def test_hand_issued_loads_are_not_read_before_their_wait(tmp_path):
-    out = tmp_path / "fused_loss.s"
+def _assembly(source, tmp_path):
+    out = tmp_path / (source + ".s")
     subprocess.run(["hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature",
                     "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-S",
-                    "--cuda-device-only", "-o", str(out), os.path.join(CSRC, "fused_loss.hip")],
+                    "--cuda-device-only", "-o", str(out), os.path.join(CSRC, source)],
                    check=True, capture_output=True)
-    text = out.read_text()
+    return out.read_text()
+
+
+def _registers(text):
+    out = set()
+    for kind, one, lo, hi in re.findall(r"\b([va])(?:(\d+)\b|\[(\d+):(\d+)\])", text):
+        out.update((kind, i) for i in range(int(one or lo), int(one or hi) + 1))
+    return out
+
+
+class _Instruction:
+    def __init__(self, text, in_asm):
+        self.text, self.in_asm = text, in_asm
+        self.op, _, rest = text.partition(" ")
+        args = [a.strip() for a in re.split(r",(?![^\[]*\])", rest)] if rest else []
+        self.target = args[0] if args else None
+        self.product = self.op.startswith("v_mfma")
+        self.slots = int(args[0], 0) + 1 if self.op == "s_nop" else 8 if self.product else 1  # (32 x 32 x 16: eight passes)
+        self.all = _registers(rest)
+        if self.product:
+            self.d, self.a, self.b, self.c = (_registers(a) for a in args[:4])
+        both = self.op.startswith(("v_permlane16_swap", "v_permlane32_swap", "v_swap"))
+        vector = self.op.startswith("v_") and not self.product
+        self.writes = _registers(" ".join(args[:2 if both else 1])) if vector else set()
+
+
+def _flow(body):
+    """(instructions, the indexes that may come next of each)"""
+    code, labels, in_asm = [], {}, False
+    for line in body:
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            in_asm = "#ASMSTART" in line
+            continue
+        text = line.split(";")[0].strip()
+        if text.endswith(":"):
+            labels[text[:-1]] = len(code)
+        elif text and not text.startswith("."):
+            code.append(_Instruction(text, in_asm))
+    after = [[] for _ in code]
+    for n, ins in enumerate(code):
+        if ins.op.startswith(("s_branch", "s_cbranch")):
+            after[n].append(labels[ins.target])
+        if ins.op not in ("s_branch", "s_endpgm") and n + 1 < len(code):
+            after[n].append(n + 1)
+    return code, after
+
+
+def _walk(start, edges, code, reach, visit):
+    """visit(instruction, issue slots between) along every path from the instructions next to one, until it says so."""
+    stack, seen = [(n, 0) for n in start], {}
+    while stack:
+        n, between = stack.pop()
+        if between < reach and seen.get(n, reach) > between:
+            seen[n] = between
+            if not visit(code[n], between):
+                stack += [(m, between + code[n].slots) for m in edges[n]]
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_inline_products_have_their_issue_slots(tmp_path):
+    """Two slots from a vector instruction that writes an operand to the product; behind it twelve to whatever else touches
+    its result (the eight passes of 32 x 32 x 16 and four), seven to a vector instruction that writes a C operand it only reads."""
+    text = _assembly("attn_kernels.hip", tmp_path)
+    counts = {}
+    for m in re.finditer(r"^_ZN3spx\d+(attn_\w+?_kernel)ILi(\d+)\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
+        code, after = _flow(m.group(0).splitlines()[1:-1])
+        before = [[] for _ in code]
+        for n, nexts in enumerate(after):
+            for s in nexts:
+                before[s].append(n)
+        for n, p in enumerate(code):
+            if not (p.product and p.in_asm):
+                continue
+            counts[m.group(1), int(m.group(2))] = counts.get((m.group(1), int(m.group(2))), 0) + 1
+            operands, held = p.a | p.b | p.c, p.c - p.d
+
+            def ahead(ins, between):
+                assert not (ins.writes & operands and between < 2), (m.group(1), ins.text, between, p.text)
+
+            def behind(ins, between):
+                assert not ins.writes & held or between >= 7, (m.group(1), p.text, between, ins.text)
+                if ins.product and ins.c == ins.d == p.d and not (ins.a | ins.b) & p.d:
+                    return True  # the next product onto it: it has a walk of its own
+                assert not ins.all & p.d or between >= 12, (m.group(1), p.text, between, ins.text)
+
+            _walk(before[n], before, code, 2, ahead)
+            _walk(after[n], after, code, 12, behind)
+    # forward at head_dim 256 (V transposed beforehand or read transposing), dQ at 256 and 64
+    assert counts == {("attn_fwd_kernel", 256): 256, ("attn_bwd_dq_kernel", 256): 96, ("attn_bwd_dq_kernel", 64): 24}
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_hand_issued_loads_are_not_read_before_their_wait(tmp_path):
+    text = _assembly("fused_loss.hip", tmp_path)
     kernels = re.findall(r"^(_ZN3spx27loss_fwd_gather_pipe_kernel\w+):", text, flags=re.M)
     assert len(kernels) == 2, kernels
     for name in kernels:
