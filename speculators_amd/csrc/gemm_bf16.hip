@@ -365,7 +365,7 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   for (; s < nslab; ++s) slab(false);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  mfma_results_ready();
+  mfma_results_ready(acc);
   if (parts > 1 && tail_mode) {
     // this part's fp32 partial of a tile of the last round: a 256 x 256 tile of its own
     float* const P = part_ws + ((int64_t)(part * n_tail + (pid - tail_first)) << 16);

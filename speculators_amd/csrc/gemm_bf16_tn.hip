@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
   if (s < nslab) slab(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  mfma_results_ready();
+  mfma_results_ready(acc);
   // epilogue: a lane holds row m of C and, per accumulator, columns 4 q + {0..3} of a 16-column block
   if constexpr (OUT >= 2) {
     float* const C = reinterpret_cast<float*>(Cv);

@@ -91,10 +91,16 @@ __device__ __forceinline__ void mfma16(f32x4& acc, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 #endif
 }
-// more wait states than the longest matrix instruction needs before its result may be read
-__device__ __forceinline__ void mfma_results_ready() {
+// More wait states than the longest matrix instruction needs before its result may be read.  The accumulators go through a
+// statement each behind them: a wait that does not name them keeps neither their readers nor their spills from coming first.
+template <int J, int I>
+__device__ __forceinline__ void mfma_results_ready(f32x4 (&acc)[J][I]) {
 #if !SPX_MFMA_BUILTIN
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int i = 0; i < I; ++i) asm volatile("" : "+a"(acc[j][i]));
 #endif
 }
 

@@ -1,7 +1,7 @@
 """Properties of the compiled code that no numerical test pins reliably.  In the pipelined gather
 kernel the registers written by the hand-issued table loads must not be read by any instruction
 before the ``s_waitcnt`` that releases them (a read before it returns whatever the register held,
-sometimes the right value).  In the attention kernels whose matrix products are inline assembly, which
+sometimes the right value).  In the attention and GEMM kernels whose matrix products are inline assembly, which
 the compiler takes for any other statement, the issue slots that such a product needs before and behind
 it must be there.  The checks compile the source to gfx950 assembly and walk it."""
 
@@ -47,7 +47,8 @@ class _Instruction:
         args = [a.strip() for a in re.split(r",(?![^\[]*\])", rest)] if rest else []
         self.target = args[0] if args else None
         self.product = self.op.startswith("v_mfma")
-        self.slots = int(args[0], 0) + 1 if self.op == "s_nop" else 8 if self.product else 1  # (32 x 32 x 16: eight passes)
+        self.passes = 8 if "32x32x16" in self.op else 4  # (16 x 16 x 32)
+        self.slots = int(args[0], 0) + 1 if self.op == "s_nop" else self.passes if self.product else 1
         self.all = _registers(rest)
         if self.product:
             self.d, self.a, self.b, self.c = (_registers(a) for a in args[:4])
@@ -89,12 +90,19 @@ def _walk(start, edges, code, reach, visit):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-def test_inline_products_have_their_issue_slots(tmp_path):
-    """Two slots from a vector instruction that writes an operand to the product; behind it twelve to whatever else touches
-    its result (the eight passes of 32 x 32 x 16 and four), seven to a vector instruction that writes a C operand it only reads."""
-    text = _assembly("attn_kernels.hip", tmp_path)
+@pytest.mark.parametrize("source,products", [
+    # forward at head_dim 256 (V transposed beforehand or read transposing), dQ at 256 and 64
+    ("attn_kernels.hip", {("attn_fwd_kernel", "256"): 256, ("attn_bwd_dq_kernel", "256"): 96, ("attn_bwd_dq_kernel", "64"): 24}),
+    # two copies of a slab of 128 products each; with and without row statistics, row factors, whole leading dimensions
+    ("gemm_bf16.hip", {("gemm_bf16_nt_kernel", "0"): 5 * 256, ("gemm_bf16_nt_kernel", "1"): 5 * 256}),
+    # three copies; four kinds of result, with and without groups
+    ("gemm_bf16_tn.hip", {("gemm_bf16_tn_kernel", str(out)): 2 * 384 for out in range(4)})])
+def test_inline_products_have_their_issue_slots(source, products, tmp_path):
+    """Two slots from a vector instruction that writes an operand to the product; behind it four more than its passes to whatever
+    else touches its result, one less than its passes to a vector instruction that writes a C operand it only reads."""
+    text = _assembly(source, tmp_path)
     counts = {}
-    for m in re.finditer(r"^_ZN3spx\d+(attn_\w+?_kernel)ILi(\d+)\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
+    for m in re.finditer(r"^_ZN3spx\w*?\d+([a-z]+_\w+?_kernel)IL[ib](\d+)\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
         code, after = _flow(m.group(0).splitlines()[1:-1])
         before = [[] for _ in code]
         for n, nexts in enumerate(after):
@@ -103,22 +111,21 @@ def test_inline_products_have_their_issue_slots(tmp_path):
         for n, p in enumerate(code):
             if not (p.product and p.in_asm):
                 continue
-            counts[m.group(1), int(m.group(2))] = counts.get((m.group(1), int(m.group(2))), 0) + 1
+            counts[m.groups()] = counts.get(m.groups(), 0) + 1
             operands, held = p.a | p.b | p.c, p.c - p.d
 
             def ahead(ins, between):
                 assert not (ins.writes & operands and between < 2), (m.group(1), ins.text, between, p.text)
 
             def behind(ins, between):
-                assert not ins.writes & held or between >= 7, (m.group(1), p.text, between, ins.text)
+                assert not ins.writes & held or between >= p.passes - 1, (m.group(1), p.text, between, ins.text)
                 if ins.product and ins.c == ins.d == p.d and not (ins.a | ins.b) & p.d:
                     return True  # the next product onto it: it has a walk of its own
-                assert not ins.all & p.d or between >= 12, (m.group(1), p.text, between, ins.text)
+                assert not ins.all & p.d or between >= p.passes + 4, (m.group(1), p.text, between, ins.text)
 
             _walk(before[n], before, code, 2, ahead)
             _walk(after[n], after, code, 12, behind)
-    # forward at head_dim 256 (V transposed beforehand or read transposing), dQ at 256 and 64
-    assert counts == {("attn_fwd_kernel", 256): 256, ("attn_bwd_dq_kernel", 256): 96, ("attn_bwd_dq_kernel", 64): 24}
+    assert counts == products
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
