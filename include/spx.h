@@ -792,6 +792,9 @@ int spx_gemm_bf16_tn_f32(const void* a, int64_t lda, const void* b, int64_t ldb,
  * holds where the product accumulates, one rounding).  workspace may be NULL (never cut); spx_gemm_tn_parts says into how
  * many parts a product is cut that has one. */
 int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T);
+/* the tiles of such a product with a workspace: 0: 256 x 256 (the kernels of the two entry points), 1: 128 x 128 by eight
+ * waves, 2: 256 x 128, 3: 64 x 128, 4: 128 x 128 by four waves, two workgroups to a compute unit */
+int spx_gemm_tn_tile(int64_t M, int64_t N, int64_t T);
 int64_t spx_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t T);
 int spx_gemm_bf16_tn_auto(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
                           int64_t N, int64_t T, int out_f32, int accumulate, void* workspace, int64_t workspace_bytes,

@@ -29,8 +29,8 @@ SIGNATURES: dict[str, list] = {
                                  _I64, _P],
     "spx_fused_vocab_loss_bwd_packed": [_I, _P, _I64, _P, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P, _P, _P,
                                         _P, _I64, _P],
-    "spx_ttt_step_reduce": [_P, _P, _P, _P, _I, _P, _I, _I64, _F, _P, _P, _P],
     "spx_block_reduce": [_P, _P, _P, _P, _I, _P, _I64, _I32, _P, _P, _P, _P, _P],
+    "spx_ttt_step_reduce": [_P, _P, _P, _P, _I, _P, _I, _I64, _F, _P, _P, _P],
     "spx_ttt_row_lo": [_P, _I, _I64, _I64, _P, _P],
     "spx_ttt_attn_workspace_bytes": [_I64, _I32, _I32, _I32, _I32],
     "spx_ttt_attn_fwd": [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _F, _P, _P,
@@ -110,6 +110,7 @@ SIGNATURES["spx_gemm_bf16_rows_graded"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _
 SIGNATURES["spx_gemm_bf16_tn"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _P]
 SIGNATURES["spx_gemm_bf16_tn_auto"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P]
 SIGNATURES["spx_gemm_tn_parts"] = [_I64, _I64, _I64]
+SIGNATURES["spx_gemm_tn_tile"] = [_I64, _I64, _I64]
 SIGNATURES["spx_gemm_tn_workspace_bytes"] = [_I64, _I64, _I64]
 SIGNATURES["spx_gemm_bf16_tn_f32"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _P]
 SIGNATURES["spx_rope_relayout_partial"] = [_P, _I64, _I32, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32,

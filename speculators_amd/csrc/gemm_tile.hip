@@ -504,6 +504,11 @@ extern "C" int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T) {
   return tile::choose_tn(M, N, T, true).parts;
 }
 
+extern "C" int spx_gemm_tn_tile(int64_t M, int64_t N, int64_t T) {
+  if (M <= 0 || N <= 0 || T <= 0) return 0;
+  return tile::choose_tn(M, N, T, true).tile;
+}
+
 extern "C" int64_t spx_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t T) {
   const int32_t parts = spx_gemm_tn_parts(M, N, T);
   return parts > 1 ? (int64_t)parts * M * N * (int64_t)sizeof(float) : 0;

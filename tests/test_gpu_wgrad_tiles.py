@@ -6,9 +6,13 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # (rows, M, N): 128 x 128 (8 waves), 256 x 128, 64 x 128, 128 x 128 (4 waves), whole rounds, tiny
-    (1537, 2056, 2040), (2665, 3080, 2048), (889, 1032, 2048), (1777, 2048, 10248), (513, 4096, 4096), (64, 8, 8),
-    (1, 136, 264), (5003, 520, 512), (8191, 264, 136), (20000, 8, 1024), (14337, 1024, 2056)]
+# (rows, M, N): (tile, in parts); 0: 256 x 256, 1: 128 x 128 by eight waves, 2: 256 x 128, 3: 64 x 128, 4: 128 x 128 by four
+CHOICE = {
+    (1537, 2056, 2040): (4, False), (2665, 3080, 2048): (2, False), (889, 1032, 2048): (3, False),
+    (1777, 2048, 10248): (2, False), (513, 4096, 4096): (0, False), (64, 8, 8): (3, False), (1, 136, 264): (3, False),
+    (831, 2664, 1288): (1, False), (5003, 520, 512): (3, True), (8191, 264, 136): (3, True), (20000, 8, 1024): (3, True),
+    (14337, 1024, 2056): (2, True), (11935, 1608, 32): (1, True), (4674, 4176, 8): (4, True)}
+SHAPES = list(CHOICE)
 
 
 @pytest.mark.parametrize("t,m,n", SHAPES)
@@ -36,9 +40,11 @@ def test_weight_gradient_against_float64(t, m, n, fp32, pad):
 
 
 def test_the_choice_falls_on_every_tile():
+    from speculators_amd import _lib
     from speculators_amd.gemm import _split_bands
 
-    assert [_split_bands(t, m, n) > 1 for t, m, n in SHAPES] == [False] * 7 + [True] * 3 + [_split_bands(14337, 1024, 2056) > 1]
+    assert {(t, m, n): (_lib.load().spx_gemm_tn_tile(m, n, t), _split_bands(t, m, n) > 1) for t, m, n in SHAPES} == CHOICE
+    assert set(CHOICE.values()) == {(0, False)} | {(tile, parts) for tile in (1, 2, 3, 4) for parts in (False, True)}
 
 
 def test_workspace_rules():
