@@ -311,27 +311,17 @@ int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows, int32_t* r
 int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail, int64_t vocab,
                    int dtype, int64_t* out, void* stream);
 
-/* Weighted masked mean and per-slot acceptance counts of a DFlash block batch:
- *   out[0] = sum_r loss[r] m_r w_r / (sum m + 1e-5),  out[1] = sum m
- *   correct[s], total[s]  (s < block_size): matches / rows with m_r != 0 at
- *   slot s = r % block_size   (compute_accuracy_multi_step, models/metrics.py:39-69)
+/* Weighted masked mean and per-slot acceptance counts of a DFlash block batch, the term's place in the loss and the step's
+ * metrics in one launch: the reduction part of models/dflash/metrics.py:20-108.  Slot of a row: s = r % block_size.
+ *   w_r = pos_weight[r] (fp32 [rows]: the D-PACE weight, losses/utils.py:64-112) or, where pos_weight is NULL,
+ *   exp(-max(s - 1, 0) / gamma), 0 at s = 0, or exp(-s / gamma) where blocks start at their anchor (from_anchor;
+ *   losses/utils.py:17-48; gamma may be any number, as there: negative, zero (weights of 0 and NaN), infinite)
  *   row_weight[r] = m_r w_r / (sum m + 1e-5)
- * `pos_weight` (fp32 [rows]) is the per-row weight: dflash_loss_decay
- * (losses/utils.py:17-48) or the D-PACE weight (losses/utils.py:64-112);
- * NULL = 1.  Replaces the reduction part of models/dflash/metrics.py:20-108. */
-int spx_block_reduce(const float* loss, const int32_t* argmax_draft,
-                     const int32_t* argmax_target, const void* mask,
-                     int mask_kind, const float* pos_weight, int64_t rows,
-                     int32_t block_size, float* out, float* correct,
-                     float* total, float* row_weight, void* stream);
-
-/* spx_block_reduce with the term's place in the loss and the step's metrics in the same launch.  pos_weight NULL: the
- * weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0, or exp(-s / gamma) where blocks start at their anchor
- * (from_anchor; losses/utils.py:17-48).  out [9 + 2 * block_size]: the two scalars of spx_block_reduce, then
- *   out[2] = *total_out = factor * out[0] (+ *total_in),  out[3], out[4] = matches, rows over the slots that count (all,
- *   or all but slot 0),  out[5] = sum of the running products of their accuracies,  out[6 .. 8] = 1,
- *   out[9 + s], out[9 + block_size + s] = matches, rows of slot s.
- * gamma may be any number, as there: negative, zero (weights of 0 and NaN), infinite. */
+ * out [9 + 2 * block_size]:
+ *   out[0] = sum_r loss[r] row_weight[r],  out[1] = sum m,  out[2] = *total_out = factor * out[0] (+ *total_in),
+ *   out[3], out[4] = matches, rows with m_r != 0 over the slots that count (all, or all but slot 0),
+ *   out[5] = sum of the running products of their accuracies,  out[6 .. 8] = 1,
+ *   out[9 + s], out[9 + block_size + s] = matches, rows of slot s (compute_accuracy_multi_step, models/metrics.py:39-69) */
 int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target, const void* mask,
                     int mask_kind, const float* pos_weight, float gamma, int from_anchor, int64_t rows,
                     int32_t block_size, float factor, const float* total_in, float* total_out, float* out,

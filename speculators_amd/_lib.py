@@ -29,7 +29,6 @@ SIGNATURES: dict[str, list] = {
                                  _I64, _P],
     "spx_fused_vocab_loss_bwd_packed": [_I, _P, _I64, _P, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P, _P, _P,
                                         _P, _I64, _P],
-    "spx_block_reduce": [_P, _P, _P, _P, _I, _P, _I64, _I32, _P, _P, _P, _P, _P],
     "spx_ttt_step_reduce": [_P, _P, _P, _P, _I, _P, _I, _I64, _F, _P, _P, _P],
     "spx_ttt_row_lo": [_P, _I, _I64, _I64, _P, _P],
     "spx_ttt_attn_workspace_bytes": [_I64, _I32, _I32, _I32, _I32],

@@ -1293,32 +1293,22 @@ __global__ __launch_bounds__(NT) void row_tokens_kernel(const int32_t* __restric
   }
 }
 
-// What spx_block_total adds to the reduction of a block batch (scalars == nullptr: nothing).
-struct BlockTotal {
-  int by_slot;            // the weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0; from_anchor: exp(-s / gamma)
-  float gamma;            // (any number: a negative one lets the weights grow)
-  int from_anchor;
-  float factor;           // the term's weight in the loss
-  const float* total_in;  // loss so far (nullptr: none)
-  float* total_out;
-  float* scalars;
-};
-
+// spx_block_total.  pos_weight == nullptr: the weight of slot s is exp(-max(s - 1, 0) / gamma), 0 at s = 0; from_anchor:
+// exp(-s / gamma).
 __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
-    const float* __restrict__ loss, const int32_t* __restrict__ pred,
-    const int32_t* __restrict__ tgt, const void* __restrict__ mask, int mask_kind,
-    const float* __restrict__ pos_weight, int64_t rows, int block_size, float* __restrict__ out,
-    float* __restrict__ correct, float* __restrict__ total, float* __restrict__ row_weight, BlockTotal bt) {
+    const float* __restrict__ loss, const int32_t* __restrict__ pred, const int32_t* __restrict__ tgt,
+    const void* __restrict__ mask, int mask_kind, const float* __restrict__ pos_weight, float gamma, int from_anchor,
+    int64_t rows, int block_size, float factor, const float* total_in, float* total_out, float* __restrict__ out,
+    float* __restrict__ row_weight) {
   __shared__ float fl[kReduceThreads / 64];
   extern __shared__ int slots[];  // [2 * block_size], and a weight per slot behind them
   float* const decay = reinterpret_cast<float*>(slots + 2 * block_size);
-  const bool by_slot = bt.by_slot;
   for (int i = threadIdx.x; i < 2 * block_size; i += kReduceThreads) slots[i] = 0;
-  if (by_slot)
+  if (!pos_weight)
     for (int i = threadIdx.x; i < block_size; i += kReduceThreads)
-      decay[i] = bt.from_anchor ? expf(-(float)i / bt.gamma) : i == 0 ? 0.f : expf(-(float)(i - 1) / bt.gamma);
+      decay[i] = from_anchor ? expf(-(float)i / gamma) : i == 0 ? 0.f : expf(-(float)(i - 1) / gamma);
   __syncthreads();
-  auto weight = [&](int64_t r) { return by_slot ? decay[r % block_size] : pos_weight ? pos_weight[r] : 1.f; };
+  auto weight = [&](int64_t r) { return pos_weight ? pos_weight[r] : decay[r % block_size]; };
   float lsum = 0.f, msum = 0.f;
   for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
     float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
@@ -1334,36 +1324,31 @@ __global__ __launch_bounds__(kReduceThreads) void block_reduce_kernel(
   lsum = block_sum_f(lsum, fl);
   msum = block_sum_f(msum, fl);
   const float inv = 1.f / (msum + 1e-5f);
-  if (threadIdx.x == 0) { out[0] = lsum * inv; out[1] = msum; }
   __syncthreads();
-  for (int i = threadIdx.x; i < block_size; i += kReduceThreads) {
-    correct[i] = (float)slots[i];
-    total[i] = (float)slots[block_size + i];
-  }
-  if (bt.scalars && threadIdx.x == 0) {
-    const float part = bt.factor * (lsum * inv), sum = bt.total_in ? *bt.total_in + part : part;
-    *bt.total_out = sum;
+  for (int i = threadIdx.x; i < 2 * block_size; i += kReduceThreads) out[9 + i] = (float)slots[i];
+  if (threadIdx.x == 0) {
+    const float part = factor * (lsum * inv), sum = total_in ? *total_in + part : part;
+    *total_out = sum;
     // the step's metrics: what a dozen one-element kernels did
     float hits = 0.f, rows_in = 0.f, run = 1.f, eal = 0.f;
-    for (int i = bt.from_anchor ? 0 : 1; i < block_size; ++i) {
+    for (int i = from_anchor ? 0 : 1; i < block_size; ++i) {
       const float c = (float)slots[i], t = (float)slots[block_size + i];
       hits += c;
       rows_in += t;
       run *= c / fmaxf(t, 1.f);
       eal += run;
     }
-    bt.scalars[0] = sum;
-    bt.scalars[1] = hits;
-    bt.scalars[2] = rows_in;
-    bt.scalars[3] = eal;
-    bt.scalars[4] = bt.scalars[5] = bt.scalars[6] = 1.f;
+    out[0] = lsum * inv;
+    out[1] = msum;
+    out[2] = sum;
+    out[3] = hits;
+    out[4] = rows_in;
+    out[5] = eal;
+    out[6] = out[7] = out[8] = 1.f;
   }
-  if (row_weight) {
-    for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
-      float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
-      float w = weight(r);
-      row_weight[r] = m * w * inv;
-    }
+  for (int64_t r = threadIdx.x; r < rows; r += kReduceThreads) {
+    const float m = mask ? mask_value(mask, mask_kind, r) : 1.f;
+    row_weight[r] = m * weight(r) * inv;
   }
 }
 
@@ -1825,40 +1810,20 @@ extern "C" int spx_row_tokens(const int32_t* known, int64_t n, const void* rows,
   return check_launch(__func__);
 }
 
-static int block_reduce(const char* fname, const float* loss, const int32_t* argmax_draft,
-                        const int32_t* argmax_target, const void* mask, int mask_kind, const float* pos_weight,
-                        int64_t rows, int32_t block_size, float* out, float* correct, float* total, float* row_weight,
-                        const BlockTotal& bt, void* stream) {
-#define SPX_REQ_FN(cond, what) do { if (!(cond)) return spx::fail_arg(fname, what); } while (0)
-  SPX_REQ_FN(rows >= 0 && rows < (1ll << 24), "0 <= rows < 2^24");
-  SPX_REQ_FN(block_size > 0 && block_size <= 4096, "0 < block_size <= 4096");
-  SPX_REQ_FN(loss && argmax_draft && argmax_target && out && correct && total, "null buffer");
-  SPX_REQ_FN(!mask || kind_ok(mask_kind), "unknown mask element kind");
-#undef SPX_REQ_FN
-  hipLaunchKernelGGL(block_reduce_kernel, dim3(1), dim3(kReduceThreads),
-                     (2 * sizeof(int) + sizeof(float)) * block_size, reinterpret_cast<hipStream_t>(stream), loss,
-                     argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
-                     correct, total, row_weight, bt);
-  return check_launch(fname);
-}
-
-extern "C" int spx_block_reduce(const float* loss, const int32_t* argmax_draft,
-                                const int32_t* argmax_target, const void* mask, int mask_kind,
-                                const float* pos_weight, int64_t rows, int32_t block_size,
-                                float* out, float* correct, float* total, float* row_weight,
-                                void* stream) {
-  return block_reduce(__func__, loss, argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
-                      correct, total, row_weight, BlockTotal{}, stream);
-}
-
 extern "C" int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_t* argmax_target,
                                const void* mask, int mask_kind, const float* pos_weight, float gamma, int from_anchor,
                                int64_t rows, int32_t block_size, float factor, const float* total_in,
                                float* total_out, float* out, float* row_weight, void* stream) {
   SPX_REQUIRE(total_out && out && row_weight, "null buffer");
-  const BlockTotal bt = {!pos_weight, gamma, from_anchor, factor, total_in, total_out, out + 2};
-  return block_reduce(__func__, loss, argmax_draft, argmax_target, mask, mask_kind, pos_weight, rows, block_size, out,
-                      out + 9, out + 9 + block_size, row_weight, bt, stream);
+  SPX_REQUIRE(rows >= 0 && rows < (1ll << 24), "0 <= rows < 2^24");
+  SPX_REQUIRE(block_size > 0 && block_size <= 4096, "0 < block_size <= 4096");
+  SPX_REQUIRE(loss && argmax_draft && argmax_target, "null buffer");
+  SPX_REQUIRE(!mask || kind_ok(mask_kind), "unknown mask element kind");
+  hipLaunchKernelGGL(block_reduce_kernel, dim3(1), dim3(kReduceThreads),
+                     (2 * sizeof(int) + sizeof(float)) * block_size, reinterpret_cast<hipStream_t>(stream), loss,
+                     argmax_draft, argmax_target, mask, mask_kind, pos_weight, gamma, from_anchor, rows, block_size,
+                     factor, total_in, total_out, out, row_weight);
+  return check_launch(__func__);
 }
 
 extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
