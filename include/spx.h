@@ -331,12 +331,17 @@ int spx_block_total(const float* loss, const int32_t* argmax_draft, const int32_
  * block_size rows: ids[r] = the anchor's token in slot 0, mask_token in the others; kv_pos [T + n_q] = positions, then
  * positions[anchor] + slot; target_row[r] = the row whose target row r predicts (its own, or the one before it);
  * aligned[r] = loss_mask of its own row, 0 for invalid anchors and (unless from_anchor) in slot 0, NaN for a valid anchor
- * whose block leaves the sequence.  Rows below 0 count from the end, each by itself.  outside (may be NULL; device or pinned host
- * memory): set to 1 where any anchor's block leaves the sequence, left as it is otherwise. */
+ * whose block leaves the sequence.  Rows below 0 count from the end, each by itself. */
 int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size, int64_t T,
                       int64_t mask_token, const int64_t* input_ids, const int64_t* positions, const void* loss_mask,
                       int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos, int64_t* target_row,
-                      float* aligned, int32_t* outside, void* stream);
+                      float* aligned, void* stream);
+/* The same; *outside (device or pinned host memory, may be NULL) is set to 1 where any anchor's block leaves the sequence,
+ * valid or not, and left as it is otherwise. */
+int spx_dflash_inputs_checked(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
+                              int64_t T, int64_t mask_token, const int64_t* input_ids, const int64_t* positions,
+                              const void* loss_mask, int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos,
+                              int64_t* target_row, float* aligned, int32_t* outside, void* stream);
 
 /* ---------------------------------------------------------------- TTT attention
  * row_lo[i] = lowest context key visible to query i: the interval form
@@ -755,6 +760,12 @@ int spx_unpack_rows(const void* packed, int64_t ld_packed, const int32_t* row_ma
 int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, const int32_t* row_map,
                            const float* row_scale, int64_t rows, int64_t total_rows,
                            int64_t cols, void* out, int64_t ld_out, void* stream);
+
+/* The same with row_scale[r] * (*scale * factor); scale: one f32 on the device (NULL: 1 and no factor).  (The rows come rounded
+ * and are rounded again here; spx_gemm_bf16_rows_graded applies the factors in front of the only rounding.) */
+int spx_unpack_rows_graded(const void* packed, int64_t ld_packed, const int32_t* row_map,
+                           const float* row_scale, const float* scale, float factor, int64_t rows,
+                           int64_t total_rows, int64_t cols, void* out, int64_t ld_out, void* stream);
 
 /* c[M, N] (+)= a[T, M]^T * b[T, N], bf16 inputs, fp32 accumulation, bf16 output:
  * the weight-gradient product of the backward of torch.nn.Linear (dW = dY^T X)

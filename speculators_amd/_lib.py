@@ -43,7 +43,8 @@ SIGNATURES["spx_vocab_loss_step_fwd"] = [_I, _P, _I64, _P, _I64, _P, _I64, _P, _
 SIGNATURES["spx_ttt_step_mean"] = [_P, _P, _I, _I64, _F, _P, _P, _P, _P]
 SIGNATURES["spx_ttt_step_total"] = [_P, _P, _P, _P, _I, _P, _I, _I64, _F, _P, _F, _P, _P, _P, _P, _P]
 SIGNATURES["spx_block_total"] = [_P, _P, _P, _P, _I, _P, _F, _I, _I64, _I32, _F, _P, _P, _P, _P, _P]
-SIGNATURES["spx_dflash_inputs"] = [_P, _P, _I64, _I32, _I64, _I64, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P]
+SIGNATURES["spx_dflash_inputs"] = [_P, _P, _I64, _I32, _I64, _I64, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P]
+SIGNATURES["spx_dflash_inputs_checked"] = [*SIGNATURES["spx_dflash_inputs"], _P]
 SIGNATURES["spx_ttt_step_terms"] = [_I32, _P, _P, _P, _I, _I64, _F, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_map"] = [_P, _I, _I64, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_lists"] = [_P, _I, _I64, _P, _P, _P, _P, _P]
@@ -93,6 +94,7 @@ SIGNATURES["spx_pack_batch"] = [_P, _I, _I64, _I64, _I64, _P, _P, _I, _P, _P, _P
 SIGNATURES["spx_gemm_bf16_nt"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]
 SIGNATURES["spx_pack_row_map"] = [_P, _P, _I64, _I64, _P, _P, _P]
 SIGNATURES["spx_unpack_rows"] = [_P, _I64, _P, _I64, _I64, _I64, _P, _I64, _P]
+SIGNATURES["spx_unpack_rows_graded"] = [_P, _I64, _P, _P, _P, _F, _I64, _I64, _I64, _P, _I64, _P]
 SIGNATURES["spx_unpack_rows_scaled"] = [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I64, _P]
 SIGNATURES["spx_vocab_loss_step_fwd_grad"] = [_I, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _I,
                                               _P, _I, _P, _I, _P, _P, _P, _I64, _P]

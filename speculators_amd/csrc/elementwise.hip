@@ -830,12 +830,15 @@ __global__ __launch_bounds__(1024) void pack_row_map_kernel(const float* __restr
 }
 
 // out[r, :] = row_map[r] >= 0 ? packed[row_map[r], :] : 0 for r < rows, 0 for rows <= r < total_rows;
-// with row_scale every live row is multiplied by row_scale[r] on its way (fp32, one rounding)
+// with row_scale every live row is multiplied by row_scale[r] on its way (fp32, one rounding) -- and with
+// scale by row_scale[r] * (*scale * factor)
 __global__ __launch_bounds__(256) void unpack_rows_kernel(const uint16_t* __restrict__ packed, int64_t ld,
                                                           const int32_t* __restrict__ row_map, int rows,
                                                           int cols8, uint16_t* __restrict__ out,
                                                           int64_t ld_out,
-                                                          const float* __restrict__ row_scale = nullptr) {
+                                                          const float* __restrict__ row_scale = nullptr,
+                                                          const float* __restrict__ scale = nullptr,
+                                                          float factor = 1.f) {
   const int r = blockIdx.x;
   const int src = r < rows ? row_map[r] : -1;
   u32x4* o = reinterpret_cast<u32x4*>(out + (int64_t)r * ld_out);
@@ -849,7 +852,7 @@ __global__ __launch_bounds__(256) void unpack_rows_kernel(const uint16_t* __rest
     for (int c = threadIdx.x; c < cols8; c += 256) o[c] = in[c];
     return;
   }
-  const float f = row_scale[r];
+  const float f = scale ? row_scale[r] * (*scale * factor) : row_scale[r];
   for (int c = threadIdx.x; c < cols8; c += 256) {
     const u32x4 v = in[c];
     u32x4 w;
@@ -889,9 +892,9 @@ extern "C" int spx_unpack_rows(const void* packed, int64_t ld_packed, const int3
   return check_launch(__func__);
 }
 
-extern "C" int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, const int32_t* row_map,
-                                      const float* row_scale, int64_t rows, int64_t total_rows, int64_t cols,
-                                      void* out, int64_t ld_out, void* stream) {
+extern "C" int spx_unpack_rows_graded(const void* packed, int64_t ld_packed, const int32_t* row_map,
+                                      const float* row_scale, const float* scale, float factor, int64_t rows,
+                                      int64_t total_rows, int64_t cols, void* out, int64_t ld_out, void* stream) {
   SPX_REQUIRE(rows > 0 && total_rows >= rows && total_rows < (1ll << 31), "rows out of range");
   SPX_REQUIRE(cols > 0 && cols % 8 == 0 && ld_packed % 8 == 0 && ld_out % 8 == 0 && ld_packed >= cols && ld_out >= cols,
               "cols and the row strides must be multiples of 8 (bf16), strides at least cols");
@@ -899,8 +902,16 @@ extern "C" int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, con
   SPX_REQUIRE(al16(packed) && al16(out), "buffers must be 16-byte aligned");
   hipLaunchKernelGGL(unpack_rows_kernel, dim3((unsigned)total_rows), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(packed), ld_packed,
-                     row_map, (int)rows, (int)(cols / 8), reinterpret_cast<uint16_t*>(out), ld_out, row_scale);
+                     row_map, (int)rows, (int)(cols / 8), reinterpret_cast<uint16_t*>(out), ld_out, row_scale, scale,
+                     factor);
   return check_launch(__func__);
+}
+
+extern "C" int spx_unpack_rows_scaled(const void* packed, int64_t ld_packed, const int32_t* row_map,
+                                      const float* row_scale, int64_t rows, int64_t total_rows, int64_t cols,
+                                      void* out, int64_t ld_out, void* stream) {
+  return spx_unpack_rows_graded(packed, ld_packed, row_map, row_scale, nullptr, 1.f, rows, total_rows, cols, out,
+                                ld_out, stream);
 }
 
 // one slot per workgroup, four workgroups per compute unit (narrow rows: one row per wave, eight)

@@ -1826,10 +1826,11 @@ extern "C" int spx_block_total(const float* loss, const int32_t* argmax_draft, c
   return check_launch(__func__);
 }
 
-extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
-                                 int64_t T, int64_t mask_token, const int64_t* input_ids, const int64_t* positions,
-                                 const void* loss_mask, int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos,
-                                 int64_t* target_row, float* aligned, int32_t* outside, void* stream) {
+extern "C" int spx_dflash_inputs_checked(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors,
+                                         int32_t block_size, int64_t T, int64_t mask_token, const int64_t* input_ids,
+                                         const int64_t* positions, const void* loss_mask, int mask_kind, int from_anchor,
+                                         int64_t* ids, int64_t* kv_pos, int64_t* target_row, float* aligned,
+                                         int32_t* outside, void* stream) {
   SPX_REQUIRE(T > 0 && T < (1ll << 30) && n_anchors >= 0 && block_size > 0 && n_anchors * block_size < (1ll << 30),
               "sizes out of range");
   SPX_REQUIRE(input_ids && positions && loss_mask && kv_pos && kind_ok(mask_kind), "null buffer or unknown mask kind");
@@ -1839,4 +1840,12 @@ extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, i
                      reinterpret_cast<hipStream_t>(stream), anchors, valid, (int)n_q, block_size, T, mask_token,
                      input_ids, positions, loss_mask, mask_kind, from_anchor, ids, kv_pos, target_row, aligned, outside);
   return check_launch(__func__);
+}
+
+extern "C" int spx_dflash_inputs(const int64_t* anchors, const uint8_t* valid, int64_t n_anchors, int32_t block_size,
+                                 int64_t T, int64_t mask_token, const int64_t* input_ids, const int64_t* positions,
+                                 const void* loss_mask, int mask_kind, int from_anchor, int64_t* ids, int64_t* kv_pos,
+                                 int64_t* target_row, float* aligned, void* stream) {
+  return spx_dflash_inputs_checked(anchors, valid, n_anchors, block_size, T, mask_token, input_ids, positions, loss_mask,
+                                   mask_kind, from_anchor, ids, kv_pos, target_row, aligned, nullptr, stream);
 }

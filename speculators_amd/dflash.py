@@ -276,7 +276,7 @@ class DFlashDraftModel(nn.Module):
         ints = torch.empty(t + 3 * n_q, device=dev, dtype=torch.int64)
         kv_pos, out_ids, idx = ints[:t + n_q], ints[t + n_q:t + 2 * n_q], ints[t + 2 * n_q:]
         aligned = torch.empty(1, n_q, device=dev, dtype=torch.float32)
-        _lib.call("spx_dflash_inputs", row(anchors.to(dev)), row(valid.to(dev), torch.bool), anchors.numel(), bs, t,
+        _lib.call("spx_dflash_inputs_checked", row(anchors.to(dev)), row(valid.to(dev), torch.bool), anchors.numel(), bs, t,
                   int(self.mask_token_id), ids, pos, mask, _lib.kind_code(mask), int(cfg.sample_from_anchor), out_ids,
                   kv_pos, idx, aligned, None if outside is None else outside.word.data_ptr(), _lib.stream_ptr(dev))
         if outside is not None:
