@@ -424,7 +424,7 @@ class _HeadStepLoss(torch.autograd.Function):
 
 def head_step_loss(op: int, x, weight, weight_t, targets, target_stats, n_rows: int, step: StepPass, mean: MeanTerm,
                    total_in=None):
-    """``head_fused_rows`` of one step with its masked mean (``mean``) added to ``total_in``: ``(total, argmax_draft,
+    """Head and loss of one step with its masked mean (``mean``) added to ``total_in``: ``(total, argmax_draft,
     argmax_target, lse_target, logits [1, T, Vd])``, the row quantities ``[n_rows]``."""
     y = _check_head(x, weight, targets, n_rows)
     t = x.shape[1]
@@ -433,10 +433,12 @@ def head_step_loss(op: int, x, weight, weight_t, targets, target_stats, n_rows: 
     return total, am_d, am_t, lse_t, logits.view(1, t, weight.shape[0])
 
 
-# From here on a step's terms share one row pass: a chunk of eight columns for each of the row pass's 512 threads.  Three
-# steps of {"ce": 0.1, "tv": 0.9}, forward and backward, head of width 2048: 4096 rows of 32000 4.24 -> 2.93 ms, of 8192 1.30 ->
-# 0.94, of 4096 1.10 -> 0.61; 512 rows 1.1 -> 0.43 - 0.52 at any width (launches).  Shorter rows would gain as well, but
-# keep the two-node form, term by term: there its results are pinned bit for bit.
+# From here on a step's terms (and the loss of anchored blocks) share one row pass: a chunk of eight columns for each of the
+# row pass's 512 threads.  Three steps of {"ce": 0.1, "tv": 0.9}, forward and backward, head of width 2048, term by term -> one
+# pass: 4096 rows of 32000 4.24 -> 2.93 ms, of 8192 1.31 -> 0.97, of 4096 1.06 -> 0.61, of 3072 1.06 -> 0.56, of 2048 1.05 -> 0.45, of
+# 1024 1.07 -> 0.42; 512 rows 1.05 -> 0.42 at any width (launches).  So the line is not where the gain ends.  It lies there
+# because shorter rows promise more: the two-node form, whose results at short rows the one-node form has to give bit for bit
+# (another order of sums in the one pass); at draft vocabularies in earnest (32000) it makes no difference.
 TERMS_MIN_VOCAB = 4096
 
 
@@ -522,8 +524,9 @@ def _check_head(x, weight, targets, n: int):
 
 
 def head_fused_rows(op: int, x, weight, weight_t, targets, target_stats=None, n_rows=None, step=None):
-    """``fused_rows`` with the frozen head in front: ``x [1, T, H]`` instead of logits.  Returns
-    ``(row_loss [1, n_rows], argmax_draft, argmax_target, lse_target, logits [1, T, Vd])``."""
+    """``fused_rows`` with the frozen head in front: ``x [1, T, H]`` instead of logits (for callers that reduce the row losses
+    themselves; the models take ``head_step_loss`` and ``head_terms_loss``).  Returns ``(row_loss [1, n_rows], argmax_draft,
+    argmax_target, lse_target, logits [1, T, Vd])``."""
     n = x.shape[1] if n_rows is None else int(n_rows)
     y = _check_head(x, weight, targets, n)
     t = x.shape[1]

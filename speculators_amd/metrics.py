@@ -107,9 +107,9 @@ def _step_views(logits, targets, loss_mask, prev_correct, ttt_step):
 
 class Head:
     """The frozen ``lm_head`` applied lazily: ``compute_metrics`` takes this in place of the logits
-    and, when the loss is a single fused HIP reduction, runs head and loss as ONE autograd node (the
+    and, when the loss is of fused HIP reductions, runs head and loss as ONE autograd node (the
     backward then skips the rows the loss mask removes in the head's input-gradient product,
-    ``losses.head_fused_rows``); otherwise the logits are made the ordinary way.  Either way
+    ``losses.head_step_loss``, ``losses.head_terms_loss``); otherwise the logits are made the ordinary way.  Either way
     ``.logits`` holds them afterwards (``[1, T, Vd]``)."""
 
     def __init__(self, x, weight, weight_t):
