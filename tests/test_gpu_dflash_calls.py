@@ -94,6 +94,14 @@ def test_a_block_that_leaves_the_sequence_is_refused(anchors, where, extra):
     _step(model, batch, [1, T - BS])  # (the last one that fits; nothing is left behind)
 
 
+def test_under_a_default_device():
+    model, batch = _model(), _batch()
+    want = _step(model, batch, [1, 17])
+    with torch.device("cuda"):
+        got = _step(model, batch, [1, 17])
+    assert torch.equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("gamma", [-3.0, float("inf"), 0.0, float("nan")])
 @pytest.mark.parametrize("from_anchor", [False, True])
 def test_decay_rates_that_are_not_positive(gamma, from_anchor):
