@@ -880,6 +880,14 @@ int spx_moe_pair_dot(const void* a, int64_t ld_a, const void* sorted, int64_t ld
                      int64_t sorted_rows, const int32_t* pos, float* out, int64_t tokens,
                      int32_t k, int64_t H, void* stream);
 
+/* Backward of the experts' SwiGLU with the router's weight in it.  hid [rows, 2 * inter]: gate and up of the sorted rows;
+ * scores: the weights of all pairs, s(p) = scores[order[p]]; dact: the gradient of s(p) * silu(gate) * up,
+ * rows of inter.  Writes dhid, the gradient of hid; act (or NULL) = s(p) * silu(gate[p]) * up[p]; dscores (or NULL; f32 or
+ * bf16), dscores[order[p]] = <dact[p], silu(gate[p]) * up[p]>. */
+int spx_moe_swiglu_bwd(const void* hid, int64_t ld_hid, const int64_t* order, const float* scores, const void* dact,
+                       int64_t ld_dact, void* dhid, int64_t ld_dhid, void* act, int64_t ld_act, void* dscores,
+                       int dscores_f32, int64_t rows, int64_t inter, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -132,6 +132,7 @@ SIGNATURES["spx_transpose_bf16"] = [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, 
 SIGNATURES["spx_moe_gather_rows"] = [_P, _I64, _I64, _P, _P, _P, _I64, _I64, _I64, _P]
 SIGNATURES["spx_moe_combine_rows"] = [_P, _I64, _I64, _P, _P, _P, _I64, _I64, _I32, _I64, _P]
 SIGNATURES["spx_moe_pair_dot"] = [_P, _I64, _P, _I64, _I64, _P, _P, _I64, _I32, _I64, _P]
+SIGNATURES["spx_moe_swiglu_bwd"] = [_P, _I64, _P, _P, _P, _I64, _P, _I64, _P, _I64, _P, _I, _I64, _I64, _P]
 SIGNATURES["spx_moe_sort_workspace_bytes"] = [_I64, _I64]
 SIGNATURES["spx_moe_sort_pairs"] = [_P, _I64, _I32, _I64, _P, _P, _P, _P, _P, _I64, _P]
 SIGNATURES["spx_gemm_auto_workspace_bytes"] = [_I, _I64, _I64, _I64, _I32]

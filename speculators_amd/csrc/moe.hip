@@ -97,6 +97,56 @@ __global__ __launch_bounds__(256) void pair_dot_kernel(const uint16_t* __restric
   if (lane == 0) out[pair] = sum;
 }
 
+// ---------------------------------------------------------------- backward of SwiGLU under the router's weight
+// An expert's output is linear in its activation, so with d[p] = W_down^T dout[token of p], not weighted yet, everything the
+// backward needs of the weight s[p] = scores[order[p]] is formed here, where a row is 512 to 768 wide, instead of on rows of
+// the hidden size: the weighted activation, which the down projection's weight gradient contracts with dout's rows as they
+// are; s[p]'s own gradient <d[p], silu(gate) * up>; and the gradient of gate and up.  Products in fp32, silu rounded to bf16
+// as in the forward, one rounding a result.  Bound by memory: 40960 rows of 512 36 us (0.21 GB); the weight in dout's rows and
+// its gradient from the outputs' rows were 74 us of reads and writes of rows of 2048 (pair_dot 33, swiglu 33, a gather of the
+// weights 6) and one rounding more of every row.
+// one wave per row
+template <typename T>
+__global__ __launch_bounds__(256) void weighted_swiglu_bwd_kernel(const uint16_t* __restrict__ hid, int64_t ld,
+                                                                  const int64_t* __restrict__ order,
+                                                                  const float* __restrict__ scores,
+                                                                  const uint16_t* __restrict__ dact, int64_t ld_d,
+                                                                  uint16_t* __restrict__ dhid, int64_t ld_dh,
+                                                                  uint16_t* __restrict__ act, int64_t ld_act,
+                                                                  T* __restrict__ dscores, int64_t rows, int inter8) {
+  const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (p >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t pair = order[p];
+  const float s = scores[pair];
+  float sum = 0.f;
+  for (int ch = lane; ch < inter8; ch += 64) {
+    float g[8], u[8], d[8], og[8], ou[8], oa[8];
+    unpack8(*reinterpret_cast<const u32x4*>(hid + p * ld + ch * 8), g);
+    unpack8(*reinterpret_cast<const u32x4*>(hid + p * ld + inter8 * 8 + ch * 8), u);
+    unpack8(*reinterpret_cast<const u32x4*>(dact + p * ld_d + ch * 8), d);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float sg = 1.f / (1.f + __expf(-g[e])), silu = g[e] * sg;
+      oa[e] = bf16_bits_to_f32(f32_to_bf16_bits(silu)) * u[e];
+      sum += d[e] * oa[e];
+      oa[e] *= s;
+      d[e] *= s;
+      ou[e] = d[e] * silu;
+      og[e] = d[e] * u[e] * (sg * (1.f + g[e] * (1.f - sg)));
+    }
+    *reinterpret_cast<u32x4*>(dhid + p * ld_dh + ch * 8) = pack8(og);
+    *reinterpret_cast<u32x4*>(dhid + p * ld_dh + inter8 * 8 + ch * 8) = pack8(ou);
+    if (act) *reinterpret_cast<u32x4*>(act + p * ld_act + ch * 8) = pack8(oa);
+  }
+  if (!dscores) return;
+  sum = wave_sum(sum);
+  if (lane == 0) {
+    if constexpr (sizeof(T) == 2) dscores[pair] = (T)f32_to_bf16_bits(sum);
+    else dscores[pair] = sum;
+  }
+}
+
 // ---------------------------------------------------------------- (token, slot) pairs sorted by expert
 // A stable counting sort in three launches.  A wave owns `per_wave` consecutive pairs (a multiple of 64): it counts
 // them per expert, the scan turns the counts into first positions (expert-major, waves in their order inside an
@@ -262,6 +312,29 @@ extern "C" int spx_moe_pair_dot(const void* a, int64_t ld_a, const void* sorted,
                      reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(a), ld_a,
                      reinterpret_cast<const uint16_t*>(sorted), ld_sorted, pos, out, pairs, (int)k, sorted_rows,
                      (int)(H / 8));
+  return check_launch(__func__);
+}
+
+extern "C" int spx_moe_swiglu_bwd(const void* hid, int64_t ld_hid, const int64_t* order, const float* scores, const void* dact,
+                                   int64_t ld_dact, void* dhid, int64_t ld_dhid, void* act, int64_t ld_act,
+                                  void* dscores, int dscores_f32, int64_t rows, int64_t inter, void* stream) {
+  SPX_REQUIRE(rows > 0 && inter > 0 && inter % 8 == 0 && inter < (1ll << 30), "rows > 0 and the width a positive multiple of 8");
+  SPX_REQUIRE(hid && order && scores && dact && dhid && al16(hid) && al16(dact) && al16(dhid) && al16(act),
+              "null or unaligned buffer");
+  SPX_REQUIRE(ld_hid % 8 == 0 && ld_dact % 8 == 0 && ld_dhid % 8 == 0 && ld_hid >= 2 * inter && ld_dhid >= 2 * inter &&
+                  ld_dact >= inter && (!act || (ld_act % 8 == 0 && ld_act >= inter)),
+              "row strides must be multiples of 8 and at least the rows' width");
+  SPX_REQUIRE((rows + 3) / 4 < (1ll << 31), "too many rows");
+  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const uint16_t *const h = reinterpret_cast<const uint16_t*>(hid), *const d = reinterpret_cast<const uint16_t*>(dact);
+  uint16_t *const o = reinterpret_cast<uint16_t*>(dhid), *const w = reinterpret_cast<uint16_t*>(act);
+  if (dscores_f32)
+    hipLaunchKernelGGL(moe::weighted_swiglu_bwd_kernel<float>, grid, block, 0, st, h, ld_hid, order, scores, d, ld_dact, o, ld_dhid, w, ld_act,
+                       reinterpret_cast<float*>(dscores), rows, (int)(inter / 8));
+  else
+    hipLaunchKernelGGL(moe::weighted_swiglu_bwd_kernel<uint16_t>, grid, block, 0, st, h, ld_hid, order, scores, d, ld_dact, o, ld_dhid, w, ld_act,
+                       reinterpret_cast<uint16_t*>(dscores), rows, (int)(inter / 8));
   return check_launch(__func__);
 }
 

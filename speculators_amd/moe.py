@@ -249,7 +249,8 @@ def sort_pairs(idx: torch.Tensor, num_experts: int):
 
 class _ExpertsMLP(torch.autograd.Function):
     """``Qwen3NextExperts.forward``: ``out[t] = sum_j scores[t, j] * down_e(silu(gate_e x_t) * up_e x_t)``,
-    ``e = idx[t, j]``, on expert-sorted rows.  The weight gradients of the uses of one forward add
+    ``e = idx[t, j]``, on expert-sorted rows.  The backward takes the scores at the activation, where a row is
+    narrow (``spx_moe_swiglu_bwd``).  The weight gradients of the uses of one forward add
     up in one buffer per weight (``Staged.grad_buffer``: fp32, or bf16 for the only use of bf16
     parameters), which the staging node hands to
     autograd once."""
@@ -266,21 +267,19 @@ class _ExpertsMLP(torch.autograd.Function):
         order, src_row, pos, off = sort_pairs(idx, e)
         rows = src_row.numel()
         st = _lib.stream_ptr(x2.device)
-        # with several uses per forward the inputs of the two products go straight into the stacks
-        # that the one weight-gradient product over all uses reads
+        # with several uses per forward the products' inputs (the down projection's: in the backward) go straight into
+        # the stacks that the one weight-gradient product over all uses reads
         stack_gu, use_gu = _ExpertStacks.use(st_gu, rows, h, i2)
         stack_dn, use_dn = _ExpertStacks.use(st_dn, rows, inter, h)
         xs = gather_rows(x2, src_row, out=None if stack_gu is None else stack_gu.x_slot(use_gu))
         hid = gemm_nt_grouped(xs, w_gu, off)
-        act = (torch.empty(rows, inter, device=x2.device, dtype=torch.bfloat16) if stack_dn is None
-               else stack_dn.x_slot(use_dn))
+        act = torch.empty(rows, inter, device=x2.device, dtype=torch.bfloat16)
         up = hid[:, inter:]
         _lib.call("spx_swiglu_rows_fwd", hid, i2, up, i2, act, inter, rows,
                   inter, st)
-        ys = gemm_nt_grouped(act, w_dn, off)
         wts = scores.float().contiguous()
-        out = combine_rows(ys, pos, wts)
-        ctx.save_for_backward(xs, hid, act, ys, pos, src_row, off, order, wts)
+        out = combine_rows(gemm_nt_grouped(act, w_dn, off), pos, wts)
+        ctx.save_for_backward(xs, hid, pos, src_row, off, order, wts)
         ctx.staged = (st_gu, st_dn)
         ctx.stacks = ((stack_gu, use_gu), (stack_dn, use_dn))
         ctx.score_dtype = scores.dtype
@@ -288,24 +287,28 @@ class _ExpertsMLP(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        xs, hid, act, ys, pos, src_row, off, order, wts = ctx.saved_tensors
+        xs, hid, pos, src_row, off, order, wts = ctx.saved_tensors
         st_gu, st_dn = ctx.staged
-        rows, inter = act.shape
-        i2 = 2 * inter
+        rows, i2 = hid.shape
+        inter = i2 // 2
         dout = dout.to(torch.bfloat16).contiguous()
         st = _lib.stream_ptr(dout.device)
-        dscores = None
-        if ctx.needs_input_grad[1]:
-            dscores = pair_dot(dout, ys, pos).to(ctx.score_dtype)
         (stack_gu, use_gu), (stack_dn, use_dn) = ctx.stacks
         want_gu, want_dn = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
-        dys = gather_rows(dout, src_row, wts.reshape(-1)[order].contiguous(),
-                          out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
+        dys = gather_rows(dout, src_row, out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
         dact = gemm_nn_grouped(dys, st_dn.w, off)
         dh = (stack_gu.dy_slot(use_gu) if stack_gu is not None and want_gu
               else torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16))
-        _lib.call("spx_swiglu_rows_bwd", hid, i2, hid[:, inter:], i2, dact, inter,
-                  dh, i2, dh[:, inter:], i2, rows, inter, st)
+        act = None
+        if want_dn:
+            act = (torch.empty(rows, inter, device=dout.device, dtype=torch.bfloat16) if stack_dn is None
+                   else stack_dn.x_slot(use_dn))
+        dscores = None
+        if ctx.needs_input_grad[1]:
+            dscores = torch.empty(wts.shape, device=dout.device, dtype=ctx.score_dtype if ctx.score_dtype == torch.bfloat16
+                                  else torch.float32)
+        _lib.call("spx_moe_swiglu_bwd", hid, i2, order, wts, dact, inter, dh, i2, act, inter, dscores,
+                  int(dscores is not None and dscores.dtype == torch.float32), rows, inter, st)
         dx = None
         if ctx.needs_input_grad[0]:
             dx = combine_rows(gemm_nn_grouped(dh, st_gu.w, off), pos, None)
@@ -321,7 +324,7 @@ class _ExpertsMLP(torch.autograd.Function):
                 buf, holds = staged.grad_buffer()
                 gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
             marks.append(staged.mark())
-        return dx, dscores, None, marks[0], marks[1], None, None
+        return dx, None if dscores is None else dscores.to(ctx.score_dtype), None, marks[0], marks[1], None, None
 
 
 def experts_mlp(x2, scores, idx, st_gu: Staged, st_dn: Staged):
