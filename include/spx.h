@@ -845,6 +845,22 @@ int spx_gemm_bf16_tn_grouped_multi(const void* a, int64_t lda, const void* b, in
                                    const int32_t* group_offsets, int64_t groups, int out_f32,
                                    int accumulate, void* stream);
 
+/* Both kinds of product with one operand's rows picked out of a larger matrix: row r of it is row src_row[r] of the
+ * src_rows x . matrix given in its place (int32 [rows] on the device; an index outside of it: a row of zeros), so that the
+ * tokens' rows need no copy in sorted order.  At most 256 rows a group on average; the matrix spans less than 2 GiB.
+ *   spx_gemm_bf16_grouped_picked:    form 0 (a b_e^T) or 1 (a b_e), rows of a picked (src_row NULL: taken as they lie).  `table`
+ *                                    is the workspace of the products above; with table_ready it holds what an earlier call
+ *                                    with the same offsets, rows and groups left there.
+ *   spx_gemm_bf16_tn_grouped_picked: rows of a (operand 0) or b (1) picked. */
+int spx_gemm_bf16_grouped_picked(int form, const void* a, int64_t lda, const int32_t* src_row, int64_t src_rows,
+                                 const void* b, int64_t ldb, int64_t b_group_stride, void* c, int64_t ldc, int64_t rows,
+                                 int64_t N, int64_t K, const int32_t* group_offsets, int64_t groups, void* table,
+                                 int64_t table_bytes, int table_ready, void* stream);
+int spx_gemm_bf16_tn_grouped_picked(const void* a, int64_t lda, const void* b, int64_t ldb, const int32_t* src_row,
+                                    int64_t src_rows, int operand, void* c, int64_t ldc, int64_t c_group_stride, int64_t M,
+                                    int64_t N, int64_t rows, const int32_t* group_offsets, int64_t groups, int out_f32,
+                                    int accumulate, void* stream);
+
 /* out[b][c][r] = in[b][r][c] for `batches` bf16 matrices of R x C (multiples of 8), row strides
  * ld_in / ld_out and batch strides in elements: the transposed copy an input-gradient product
  * reads where it runs in the NT form (of few, large tiles; the NN forms -- spx_gemm_bf16_auto form 1,

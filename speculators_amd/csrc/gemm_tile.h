@@ -104,6 +104,47 @@ struct Operand {
     }
   }
 
+  // The same with rows picked out of a larger matrix: row r of the operand is row src[r] of `base` (a number outside of
+  // 0 .. src_rows - 1: zeros).  The whole of that matrix lies below 2 GiB.
+  // SLOW = false: the operand's rows, looked up once here
+  __device__ __forceinline__ void init_picked(const uint16_t* base, int64_t ld, int rows, int len, int wave, int lane,
+                                              const int32_t* src, int src_rows) {
+    init(base, ld, rows, len, wave, lane);
+    rsrc = make_rsrc(base, len > 0 ? (uint32_t)((((int64_t)src_rows - 1) * ld + len) * 2) : 0u);
+    const int lrow = lane >> 3;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int r = (wave * kLoads + j) * 8 + lrow;
+      const int from = r < rows ? src[r] : -1;
+      off[j] = (uint32_t)from < (uint32_t)src_rows ? off[j] + (int)((int64_t)(from - r) * ld * 2) : kOob;
+    }
+  }
+  // SLOW = true: the contraction's rows, looked up slab by slab (`pick`, a slab ahead of its loads)
+  __device__ __forceinline__ void init_picked_slow(const uint16_t* base, int64_t ld, int cols, int wave, int lane, int src_rows) {
+    init(base, ld, cols, 1, wave, lane);
+    rsrc = make_rsrc(base, (uint32_t)((((int64_t)src_rows - 1) * ld + min(cols, kR)) * 2));
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j)
+      if (off[j] != kOob) off[j] -= slab_row(j, wave, lane) * row_bytes;  // (the column's part alone)
+  }
+  __device__ __forceinline__ static int slab_row(int j, int wave, int lane) {
+    constexpr int kPerLoad = 1024 / (kR * 2);
+    return kPerLoad * (wave * kLoads + j) + lane / (kR * 2 / 16);
+  }
+  __device__ __forceinline__ void pick(int (&rows)[kLoads], const int32_t* src, int src_rows, int k0, int len, int wave,
+                                       int lane) const {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int k = k0 + slab_row(j, wave, lane);
+      const int from = k < len ? src[k] : -1;
+      rows[j] = (uint32_t)from < (uint32_t)src_rows ? from : -1;
+    }
+  }
+  __device__ __forceinline__ void load_picked(int j, uint32_t lds, const int (&rows)[kLoads], int wave) const {
+    const bool in = rows[j] >= 0 && off[j] != kOob;
+    load_to_lds16<0>(rsrc, lds + (wave * kLoads + j) * 1024, in ? off[j] + rows[j] * row_bytes : kOob, 0);
+  }
+
   // wave-load j of the slab at contraction index k0 into the LDS slab at `lds` (this operand's base)
   __device__ __forceinline__ void load(int j, uint32_t lds, int k0, int len, int wave) const {
     const uint32_t dst = lds + (wave * kLoads + j) * 1024;
@@ -156,13 +197,18 @@ struct Params {
   const int32_t* group_off;     // grouped: group boundaries
   const int32_t* m_live;        // how many leading rows of A count (device; null: all M)
   int64_t group_stride;         // elements between the groups' B (NT / NN) or C (TN)
+  const int32_t* src;           // PICK: where each of the operand's rows lies in the matrix it is picked from ...
+  int src_rows;                 // ... and that matrix's rows
   RowGrade grade;               // GRADE: what the rows are multiplied by
 };
 
 // OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C.  STREAM: non-temporal stores (OUT 0 and 2).  GRADE: rows
-// multiplied by their factors on the way to their rounding (OUT 0; of a product in parts the pass that adds them does it)
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE>
+// multiplied by their factors on the way to their rounding (OUT 0; of a product in parts the pass that adds them does it).
+// PICK (grouped): the rows of A (1) or B (2) -- of the contraction, where that is the slow index -- are those of a larger
+// matrix that p.src names
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE, int PICK>
 __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p) {
+  static_assert(PICK == 0 || (AT ? BT && STAGES == 1 : PICK == 1), "picked rows: A of the NT and NN forms, one slab of TN");
   constexpr int kWaves = WM * WN, kMI = TM / WM / 16, kNI = TN / WN / 16;
   using OA = Operand<TM, kWaves, AT>;
   using OB = Operand<TN, kWaves, BT>;
@@ -217,8 +263,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   if (AT && p.group_off) {  // grouped TN: blockIdx.y = group, the contraction runs over its rows
     const int e = blockIdx.y;
     const int t0 = min(max(p.group_off[e], 0), p.K), t1 = min(max(p.group_off[e + 1], t0), p.K);
-    A += (int64_t)t0 * p.lda;
-    B += (int64_t)t0 * p.ldb;
+    if (PICK != 1) A += (int64_t)t0 * p.lda;
+    if (PICK != 2) B += (int64_t)t0 * p.ldb;
+    if (PICK) p.src += t0;
     K = t1 - t0;
     C = reinterpret_cast<uint8_t*>(C) + (int64_t)e * p.group_stride * (OUT >= 2 ? 4 : 2);
     if ((OUT & 1) && K == 0) return;
@@ -233,8 +280,11 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
 
   OA oa;
   OB ob;
-  oa.init(AT ? A + m0 : A + (int64_t)m0 * p.lda, p.lda, M - m0, K, wave, lane);
-  ob.init(BT ? B + n0 : B + (int64_t)n0 * p.ldb, p.ldb, p.N - n0, K, wave, lane);
+  if constexpr (PICK == 1 && AT) oa.init_picked_slow(A + m0, p.lda, M - m0, wave, lane, p.src_rows);
+  else if constexpr (PICK == 1) oa.init_picked(A, p.lda, M - m0, K, wave, lane, p.src + m0, p.src_rows);
+  else oa.init(AT ? A + m0 : A + (int64_t)m0 * p.lda, p.lda, M - m0, K, wave, lane);
+  if constexpr (PICK == 2) ob.init_picked_slow(B + n0, p.ldb, p.N - n0, wave, lane, p.src_rows);
+  else ob.init(BT ? B + n0 : B + (int64_t)n0 * p.ldb, p.ldb, p.N - n0, K, wave, lane);
   const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
   const uint32_t a_rd = OA::read_base(lds0, wm, lane), b_rd = OB::read_base(lds0 + OA::kBytes, wn, lane);
 
@@ -247,9 +297,20 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   const int nslab = (K + kTK - 1) / kTK;
   int ld_k = 0;  // contraction index of the slab being loaded
   uint32_t ld_at = lds0;
+  constexpr int kPick = AT ? PICK : 0;
+  int picked[kPick == 1 ? OA::kLoads : OB::kLoads];  // rows of the slab that is loaded next
+  auto pick = [&](int k0) __attribute__((always_inline)) {
+    if constexpr (kPick == 1) oa.pick(picked, p.src, p.src_rows, k0, K, wave, lane);
+    else if constexpr (kPick == 2) ob.pick(picked, p.src, p.src_rows, k0, K, wave, lane);
+  };
   auto issue_one = [&](int l) __attribute__((always_inline)) {
-    if (l < OA::kLoads) oa.load(l, ld_at, ld_k, K, wave);
-    else ob.load(l - OA::kLoads, ld_at + OA::kBytes, ld_k, K, wave);
+    if (l < OA::kLoads) {
+      if constexpr (kPick == 1) oa.load_picked(l, ld_at, picked, wave);
+      else oa.load(l, ld_at, ld_k, K, wave);
+    } else {
+      if constexpr (kPick == 2) ob.load_picked(l - OA::kLoads, ld_at + OA::kBytes, picked, wave);
+      else ob.load(l - OA::kLoads, ld_at + OA::kBytes, ld_k, K, wave);
+    }
   };
   auto next_load = [&]() __attribute__((always_inline)) {
     ld_k += kTK;
@@ -291,8 +352,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
           acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[j][i], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     };
+    pick(0);
 #pragma unroll
     for (int l = 0; l < kL; ++l) issue_one(l);
+    if (nslab > 1) pick(kTK);
     for (int s = 0; s < nslab; ++s) {
       wait_vmcnt<0>();
       __builtin_amdgcn_s_barrier();
@@ -314,6 +377,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
         ld_k += kTK;
 #pragma unroll
         for (int l = 0; l < kL; ++l) issue_one(l);
+        if (s + 2 < nslab) pick(ld_k + kTK);
       }
       __builtin_amdgcn_sched_barrier(0);
       products();

@@ -57,14 +57,16 @@ __global__ __launch_bounds__(256) void group_tiles_kernel(const int32_t* __restr
 }
 
 constexpr int kCus = 256;
+constexpr int kPickRows = 256;  // rows a group on average up to which the grouped products take their rows picked
 
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE = false>
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE = false,
+          int PICK = 0>
 static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
   constexpr int kSmem = (TM + TN) * kTK * 2 * STAGES;
   static std::atomic<uint64_t> lds_set;
-  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE>;
+  auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE, PICK>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmem, lds_set, fname)) return rc;
-  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE>),
+  hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE, PICK>),
                      dim3((unsigned)(p.tiles_m * p.tiles_n * p.parts), (unsigned)groups_y), dim3(64 * WM * WN), kSmem,
                      st, p);
   return check_launch(fname);
@@ -75,22 +77,26 @@ static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
 static int64_t table_entries(int64_t rows, int64_t groups, int tm) { return (rows + tm - 1) / tm + groups; }
 
 // Grouped product over the rows of A: c[r, :] = a[r, :] b_e^T (BT = false, b_e [N, K]) or a[r, :] b_e (BT = true,
-// b_e [K, N]).
+// b_e [K, N]).  src: where the rows of A lie in a matrix of src_rows (null: in order); table_ready: the workspace holds the
+// table of tile rows already.
 template <bool BT>
 static int grouped_rows(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb,
                         int64_t b_group_stride, void* c, int64_t ldc, int64_t rows, int64_t N, int64_t K,
-                        const int32_t* group_off, int64_t groups, void* workspace, hipStream_t st) {
+                        const int32_t* group_off, int64_t groups, void* workspace, hipStream_t st,
+                        const int32_t* src = nullptr, int64_t src_rows = 0, bool table_ready = false) {
   // Rows a group on average: above 256 the taller tile reads the group's weights half as often (64 groups of 1024 rows,
   // K 2048 -> N 1536, 768 -> 2048: NT 413 -> 404 us, 254 -> 240; of 4096: 1568 -> 1385, 978 -> 876; of 256, 512 groups:
   // 1054 -> 1084, 634 -> 641; NN 220 -> 220, 457 -> 425; of 256: 550 -> 584, 1095 -> 1095).
-  const bool wide_m = rows > 256 * groups;
+  const bool wide_m = rows > kPickRows * groups;
   const int tm = wide_m ? 256 : 128;
   const int64_t max_tiles = table_entries(rows, groups, tm), tiles_n = (N + 255) / 256;
   SPX_REQ_FN(max_tiles * tiles_n < (1ll << 31), "too many tiles");
   int32_t* const tab = reinterpret_cast<int32_t*>(workspace);
-  hipLaunchKernelGGL(group_tiles_kernel, dim3(1), dim3(256), 0, st, group_off, (int)groups, (int)rows, tm,
-                     (int)max_tiles, tab);
-  if (int rc = check_launch(fname)) return rc;
+  if (!table_ready) {
+    hipLaunchKernelGGL(group_tiles_kernel, dim3(1), dim3(256), 0, st, group_off, (int)groups, (int)rows, tm,
+                       (int)max_tiles, tab);
+    if (int rc = check_launch(fname)) return rc;
+  }
   Params p{};
   p.A = reinterpret_cast<const uint16_t*>(a);
   p.B = reinterpret_cast<const uint16_t*>(b);
@@ -99,12 +105,17 @@ static int grouped_rows(const char* fname, const void* a, int64_t lda, const voi
   p.M = (int)rows; p.N = (int)N; p.K = (int)K;
   p.tiles_m = (int)max_tiles; p.tiles_n = (int)tiles_n; p.parts = 1;
   p.tile_tab = tab; p.group_off = group_off; p.group_stride = b_group_stride;
+  p.src = src; p.src_rows = (int)src_rows;
   if (wide_m) return launch<256, 256, 2, 4, 2, 2, false, BT, 0, true>(fname, p, 1, st);
   // A short contraction is mostly start and end of a tile: two workgroups with one slab each cover them, three slabs of
   // one workgroup do not -- where there are tiles for two (512 groups of 80 rows: K 512 -> N 2048 NT 247 -> 236 us, K 1024
   // -> 2048 NN 430 -> 409; 64 groups of 88 rows: 34 -> 35, 57 -> 66; K 2048: 432 / 431 NT, 234 -> 245 NN)
-  if (K <= 1024 && groups * tiles_n >= 4 * kCus) return launch<128, 256, 2, 4, 1, 4, false, BT, 0, true>(fname, p, 1, st);
-  return launch<128, 256, 2, 4, 3, 2, false, BT, 0, true>(fname, p, 1, st);
+  const bool short_k = K <= 1024 && groups * tiles_n >= 4 * kCus;
+  if (src)
+    return short_k ? launch<128, 256, 2, 4, 1, 4, false, BT, 0, true, false, 1>(fname, p, 1, st)
+                   : launch<128, 256, 2, 4, 3, 2, false, BT, 0, true, false, 1>(fname, p, 1, st);
+  return short_k ? launch<128, 256, 2, 4, 1, 4, false, BT, 0, true>(fname, p, 1, st)
+                 : launch<128, 256, 2, 4, 3, 2, false, BT, 0, true>(fname, p, 1, st);
 }
 
 int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t b_group_stride,
@@ -122,21 +133,21 @@ int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int
                              reinterpret_cast<hipStream_t>(stream));
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int MINB>
+template <int TM, int TN, int WM, int WN, int STAGES, int MINB, int PICK = 0>
 static int launch_tn_tile(const char* fname, Params p, int64_t groups, int out, hipStream_t st) {
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
   switch (out) {
-    case 0: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 0, true>(fname, p, (int)groups, st);
-    case 1: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 1, false>(fname, p, (int)groups, st);
-    case 2: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 2, true>(fname, p, (int)groups, st);
-    default: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 3, false>(fname, p, (int)groups, st);
+    case 0: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 0, true, false, PICK>(fname, p, (int)groups, st);
+    case 1: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 1, false, false, PICK>(fname, p, (int)groups, st);
+    case 2: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 2, true, false, PICK>(fname, p, (int)groups, st);
+    default: return launch<TM, TN, WM, WN, STAGES, MINB, true, true, 3, false, false, PICK>(fname, p, (int)groups, st);
   }
 }
 
 int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                int64_t c_group_stride, int64_t M, int64_t N, int64_t rows, const int32_t* group_off, int64_t groups,
-               int out_f32, int accumulate, void* stream) {
+               int out_f32, int accumulate, void* stream, const int32_t* src, int64_t src_rows, int operand) {
   Params p{};
   p.A = reinterpret_cast<const uint16_t*>(a);
   p.B = reinterpret_cast<const uint16_t*>(b);
@@ -151,6 +162,12 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
   // another.  (1024, 2048 results; 256 x 256 with whole lines / 128 x 128: 512 groups of 10 rows 460 / 350 us, of 80
   // 546 / 467, of 256 (1536 columns) 1428 / 1356; 64 groups of 1024 rows 439 / 440 and, 2048 x 768, 250 / 269; of 2048
   // rows 522 / 752.)
+  if (src) {
+    p.src = src;
+    p.src_rows = (int)src_rows;
+    return operand ? launch_tn_tile<128, 128, 2, 2, 1, 4, 2>(fname, p, groups, out, st)
+                   : launch_tn_tile<128, 128, 2, 2, 1, 4, 1>(fname, p, groups, out, st);
+  }
   return rows <= 512 * groups ? launch_tn_tile<128, 128, 2, 2, 1, 4>(fname, p, groups, out, st)
                               : launch_tn_tile<256, 256, 2, 4, 2, 2>(fname, p, groups, out, st);
 }
@@ -402,6 +419,53 @@ extern "C" int spx_gemm_bf16_nn_grouped(const void* a, int64_t lda, const void* 
              "256 rows of a and one group of b must span less than 2 GiB (32-bit offsets)");
   return tile::grouped_rows<true>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups,
                                   workspace, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int spx_gemm_bf16_grouped_picked(int form, const void* a, int64_t lda, const int32_t* src_row,
+                                            int64_t src_rows, const void* b, int64_t ldb, int64_t b_group_stride, void* c,
+                                            int64_t ldc, int64_t rows, int64_t N, int64_t K, const int32_t* group_offsets,
+                                            int64_t groups, void* table, int64_t table_bytes, int table_ready,
+                                            void* stream) {
+  const char* fname = __func__;
+  SPX_REQ_FN(form == 0 || form == 1, "form must be 0 (a b^T) or 1 (a b)");
+  SPX_REQ_FN(rows > 0 && N > 0 && K > 0, "rows, N, K must be positive");
+  SPX_REQ_FN(rows < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "dimension too large");
+  SPX_REQ_FN(a && b && c, "null buffer");
+  SPX_REQ_FN(groups > 0 && groups < (1 << 24) && rows <= tile::kPickRows * groups, "up to 256 rows a group on average");
+  SPX_REQ_FN(group_offsets && table, "null group offsets or table");
+  SPX_REQ_FN(table_bytes >= spx_gemm_grouped_workspace_bytes(rows, groups), "table too small");
+  SPX_REQ_FN(((uintptr_t)table) % 4 == 0 && b_group_stride % 8 == 0 && b_group_stride >= 0,
+             "unaligned table or group stride");
+  SPX_REQ_FN(K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && (!form || N % 8 == 0),
+             "K, lda, ldb (and N of a b) must be multiples of 8");
+  SPX_REQ_FN(lda >= K && ldb >= (form ? N : K) && ldc >= N, "leading dimension too small");
+  SPX_REQ_FN(((uintptr_t)a | (uintptr_t)b) % 16 == 0, "a and b must be 16-byte aligned");
+  SPX_REQ_FN((256 * lda + K) * 2 < 0x7ffffff0ll && (form ? (K + 4 * tile::kTK) * ldb : 256 * ldb + K) * 2 < 0x7ffffff0ll,
+             "256 rows of a and of one group of b must span less than 2 GiB (32-bit offsets)");
+  SPX_REQ_FN(!src_row || (src_rows > 0 && src_rows * lda * 2 < 0x7ffffff0ll),
+             "the matrix that rows are picked from must have rows and span less than 2 GiB (32-bit offsets)");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return form ? tile::grouped_rows<true>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups, table,
+                                         st, src_row, src_rows, table_ready != 0)
+              : tile::grouped_rows<false>(fname, a, lda, b, ldb, b_group_stride, c, ldc, rows, N, K, group_offsets, groups, table,
+                                          st, src_row, src_rows, table_ready != 0);
+}
+
+extern "C" int spx_gemm_bf16_tn_grouped_picked(const void* a, int64_t lda, const void* b, int64_t ldb, const int32_t* src_row,
+                                               int64_t src_rows, int operand, void* c, int64_t ldc, int64_t c_group_stride,
+                                               int64_t M, int64_t N, int64_t rows, const int32_t* group_offsets,
+                                               int64_t groups, int out_f32, int accumulate, void* stream) {
+  const char* fname = __func__;
+  if (int rc = tile::tn_check(fname, a, lda, b, ldb, c, ldc, M, N, rows)) return rc;
+  SPX_REQ_FN(group_offsets && groups > 0 && groups < 65536, "null group offsets or a group count outside 1 .. 65535");
+  SPX_REQ_FN(c_group_stride >= (M - 1) * ldc + N, "groups of c overlap");
+  SPX_REQ_FN(c_group_stride % (out_f32 ? 4 : 8) == 0, "the groups of c must be 16-byte aligned among each other");
+  SPX_REQ_FN(rows <= tile::kPickRows * groups, "up to 256 rows a group on average");
+  SPX_REQ_FN(operand == 0 || operand == 1, "operand must be 0 (a) or 1 (b)");
+  SPX_REQ_FN(src_row && src_rows > 0 && src_rows * (operand ? ldb : lda) * 2 < 0x7ffffff0ll,
+             "the matrix that rows are picked from must have rows and span less than 2 GiB (32-bit offsets)");
+  return tile::grouped_tn(fname, a, lda, b, ldb, c, ldc, c_group_stride, M, N, rows, group_offsets, groups, out_f32, accumulate,
+                          stream, src_row, src_rows, operand);
 }
 
 // whether the contraction of a product may be cut: the partials are stored in groups of four columns

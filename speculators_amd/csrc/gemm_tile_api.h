@@ -28,7 +28,8 @@ int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int
                void* workspace, void* stream);
 int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                int64_t c_group_stride, int64_t M, int64_t N, int64_t rows, const int32_t* group_off, int64_t groups,
-               int out_f32, int accumulate, void* stream);
+               int out_f32, int accumulate, void* stream, const int32_t* src = nullptr, int64_t src_rows = 0,
+               int operand = 0);
 
 // the argument rules of every weight-gradient product (gemm_bf16_tn.hip)
 int tn_check(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, const void* c, int64_t ldc, int64_t M,

@@ -247,6 +247,57 @@ def sort_pairs(idx: torch.Tensor, num_experts: int):
     return order, src_row, pos.view(t, k), offsets
 
 
+PICK_ROWS = 256  # rows a group on average that the picked products take
+PICK_BYTES = 0x7ffffff0
+
+
+class _Picked:
+    """The expert products on tokens' rows as they lie: row r of an operand is row ``src_row[r]`` of the tokens'
+    matrix (a few MB that the caches hold), looked up by the product's own loads.  The four products of a forward and
+    backward share one table of tile rows.
+
+    On copies in sorted order / picked, us: 4096 tokens, top 10 of 512 experts of 512 (a copy: 48), forward 414 / 399,
+    input gradient 238 / 223, weight gradients 612 + 321 / 520 + 291; 1500, 8 of 128 (17): 141 / 134, 79 / 76, 163 + 85
+    / 127 + 69; 2048, 8 of 64 of 768, 256 rows each (21): 141 / 140, 74 / 66, 181 + 98 / 168 + 91; 12000, 10 of 512, 234
+    rows each (141): 672 / 637, 358 / 343, 946 + 465 / 965 + 471."""
+
+    def __init__(self, src_row, off):
+        self.src_row, self.off, self.table = src_row, off, None
+
+    @staticmethod
+    def takes(x2, rows: int, experts: int) -> bool:
+        """Whether ``x2``'s rows are picked (else they are copied into sorted order first): few rows an expert (above 256
+        the products take tall tiles, are bound by their arithmetic and have no picked form) and a matrix that 32-bit
+        offsets reach."""
+        return 0 < rows <= PICK_ROWS * experts and x2.shape[0] * x2.shape[1] * 2 < PICK_BYTES
+
+    def rows_of(self, form: int, a, b, picked: bool):
+        """``a[src_row]`` (``picked``) or ``a`` times every expert's ``b.T`` (form 0) or ``b`` (form 1)."""
+        groups, n, k = b.shape if form == 0 else (b.shape[0], b.shape[2], b.shape[1])
+        rows = self.src_row.numel()
+        if (b.dtype != torch.bfloat16 or a.shape[1] != k or not b.is_contiguous() or self.off.numel() != groups + 1
+                or (not picked and a.shape[0] != rows)):
+            raise ValueError(f"shape mismatch: a {tuple(a.shape)} b {tuple(b.shape)} (b bf16, contiguous)")
+        native = _lib.native()
+        nbytes = int(native.spx_gemm_grouped_workspace_bytes(rows, groups))
+        ready = self.table is not None
+        if not ready:
+            self.table = torch.empty(nbytes // 4, device=a.device, dtype=torch.int32)
+        out = torch.empty(rows, n, device=a.device, dtype=torch.bfloat16)
+        _lib.call("spx_gemm_bf16_grouped_picked", form, a, a.stride(0), self.src_row if picked else None, a.shape[0], b,
+                  b.stride(1), b.stride(0), out, n, rows, n, k, self.off, groups, self.table, nbytes, int(ready),
+                  _lib.stream_ptr(a.device))
+        return out
+
+    def weight_gradient(self, a, b, operand: int, out, accumulate: bool):
+        """``out[e] (+)= a[rows of e].T @ b[rows of e]``, the rows of a (operand 0) or b (1) picked."""
+        groups, m, n = out.shape
+        src = (a, b)[operand]
+        _lib.call("spx_gemm_bf16_tn_grouped_picked", a, a.stride(0), b, b.stride(0), self.src_row, src.shape[0], operand, out, n,
+                  m * n, m, n, self.src_row.numel(), self.off, groups, int(out.dtype == torch.float32), int(accumulate),
+                  _lib.stream_ptr(a.device))
+
+
 class _ExpertsMLP(torch.autograd.Function):
     """``Qwen3NextExperts.forward``: ``out[t] = sum_j scores[t, j] * down_e(silu(gate_e x_t) * up_e x_t)``,
     ``e = idx[t, j]``, on expert-sorted rows.  The backward takes the scores at the activation, where a row is
@@ -271,15 +322,24 @@ class _ExpertsMLP(torch.autograd.Function):
         # the stacks that the one weight-gradient product over all uses reads
         stack_gu, use_gu = _ExpertStacks.use(st_gu, rows, h, i2)
         stack_dn, use_dn = _ExpertStacks.use(st_dn, rows, inter, h)
-        xs = gather_rows(x2, src_row, out=None if stack_gu is None else stack_gu.x_slot(use_gu))
-        hid = gemm_nt_grouped(xs, w_gu, off)
+        picked = None
+        if stack_gu is None and stack_dn is None and _Picked.takes(x2, rows, e):
+            if x2.stride(1) != 1:
+                x2 = x2.contiguous()
+            picked, xs = _Picked(src_row, off), x2
+            hid = picked.rows_of(0, x2, w_gu, True)
+        else:
+            xs = gather_rows(x2, src_row, out=None if stack_gu is None else stack_gu.x_slot(use_gu))
+            hid = gemm_nt_grouped(xs, w_gu, off)
         act = torch.empty(rows, inter, device=x2.device, dtype=torch.bfloat16)
         up = hid[:, inter:]
         _lib.call("spx_swiglu_rows_fwd", hid, i2, up, i2, act, inter, rows,
                   inter, st)
         wts = scores.float().contiguous()
-        out = combine_rows(gemm_nt_grouped(act, w_dn, off), pos, wts)
+        ys = gemm_nt_grouped(act, w_dn, off) if picked is None else picked.rows_of(0, act, w_dn, False)
+        out = combine_rows(ys, pos, wts)
         ctx.save_for_backward(xs, hid, pos, src_row, off, order, wts)
+        ctx.picked = picked
         ctx.staged = (st_gu, st_dn)
         ctx.stacks = ((stack_gu, use_gu), (stack_dn, use_dn))
         ctx.score_dtype = scores.dtype
@@ -295,8 +355,13 @@ class _ExpertsMLP(torch.autograd.Function):
         st = _lib.stream_ptr(dout.device)
         (stack_gu, use_gu), (stack_dn, use_dn) = ctx.stacks
         want_gu, want_dn = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
-        dys = gather_rows(dout, src_row, out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
-        dact = gemm_nn_grouped(dys, st_dn.w, off)
+        picked = ctx.picked
+        if picked is not None:
+            dys = dout
+            dact = picked.rows_of(1, dout, st_dn.w, True)
+        else:
+            dys = gather_rows(dout, src_row, out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
+            dact = gemm_nn_grouped(dys, st_dn.w, off)
         dh = (stack_gu.dy_slot(use_gu) if stack_gu is not None and want_gu
               else torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16))
         act = None
@@ -311,10 +376,11 @@ class _ExpertsMLP(torch.autograd.Function):
                   int(dscores is not None and dscores.dtype == torch.float32), rows, inter, st)
         dx = None
         if ctx.needs_input_grad[0]:
-            dx = combine_rows(gemm_nn_grouped(dh, st_gu.w, off), pos, None)
+            dxs = gemm_nn_grouped(dh, st_gu.w, off) if picked is None else picked.rows_of(1, dh, st_gu.w, False)
+            dx = combine_rows(dxs, pos, None)
         marks = []
-        for need, staged, dy2, x2, stack, use in ((want_gu, st_gu, dh, xs, stack_gu, use_gu),
-                                                 (want_dn, st_dn, dys, act, stack_dn, use_dn)):
+        for need, staged, dy2, x2, stack, use, tokens in ((want_gu, st_gu, dh, xs, stack_gu, use_gu, 1),
+                                                         (want_dn, st_dn, dys, act, stack_dn, use_dn, 0)):
             if not need:
                 marks.append(None)
                 continue
@@ -322,7 +388,10 @@ class _ExpertsMLP(torch.autograd.Function):
                 stack.record(use, off)  # the product runs once, over all uses, in the staging node
             else:
                 buf, holds = staged.grad_buffer()
-                gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
+                if picked is not None:
+                    picked.weight_gradient(dy2, x2, tokens, buf, holds)
+                else:
+                    gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
             marks.append(staged.mark())
         return dx, None if dscores is None else dscores.to(ctx.score_dtype), None, marks[0], marks[1], None, None
 
