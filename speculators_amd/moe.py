@@ -374,15 +374,13 @@ class _ExpertsMLP(torch.autograd.Function):
                                   else torch.float32)
         _lib.call("spx_moe_swiglu_bwd", hid, i2, order, wts, dact, inter, dh, i2, act, inter, dscores,
                   int(dscores is not None and dscores.dtype == torch.float32), rows, inter, st)
-        dx = None
-        if ctx.needs_input_grad[0]:
-            dxs = gemm_nn_grouped(dh, st_gu.w, off) if picked is None else picked.rows_of(1, dh, st_gu.w, False)
-            dx = combine_rows(dxs, pos, None)
-        marks = []
-        for need, staged, dy2, x2, stack, use, tokens in ((want_gu, st_gu, dh, xs, stack_gu, use_gu, 1),
-                                                         (want_dn, st_dn, dys, act, stack_dn, use_dn, 0)):
+        # The weight gradients before the input gradient, the narrow operand first: act and dh have just been written (126 MB
+        # for 40960 rows) and are read out of the memory-side cache, which the input gradient's pass over the weights (2.1 GB)
+        # would leave empty.  4096 tokens, top 10 of 512 experts: 621 + 322 -> 537 + 276 us, the pass 2458 -> 2310.
+        marks = {}
+        for need, staged, dy2, x2, stack, use, tokens in ((want_dn, st_dn, dys, act, stack_dn, use_dn, 0),
+                                                         (want_gu, st_gu, dh, xs, stack_gu, use_gu, 1)):
             if not need:
-                marks.append(None)
                 continue
             if stack is not None:
                 stack.record(use, off)  # the product runs once, over all uses, in the staging node
@@ -392,8 +390,12 @@ class _ExpertsMLP(torch.autograd.Function):
                     picked.weight_gradient(dy2, x2, tokens, buf, holds)
                 else:
                     gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
-            marks.append(staged.mark())
-        return dx, None if dscores is None else dscores.to(ctx.score_dtype), None, marks[0], marks[1], None, None
+            marks[staged] = staged.mark()
+        dx = None
+        if ctx.needs_input_grad[0]:
+            dxs = gemm_nn_grouped(dh, st_gu.w, off) if picked is None else picked.rows_of(1, dh, st_gu.w, False)
+            dx = combine_rows(dxs, pos, None)
+        return dx, None if dscores is None else dscores.to(ctx.score_dtype), None, marks.get(st_gu), marks.get(st_dn), None, None
 
 
 def experts_mlp(x2, scores, idx, st_gu: Staged, st_dn: Staged):
