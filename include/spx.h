@@ -306,6 +306,37 @@ int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row
 int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
                        int32_t* row_of, int32_t* zero3, void* stream);
 
+/* Loss, acceptance chain, draft tokens and unit-weight logits gradient of ALL steps of a TTT loop (kl or ce; bf16; vocab a
+ * multiple of 8, at most 32768; 1 .. SPX_LOSS_STEPS_MAX steps, no more than rows): draft row t of step k meets target row
+ * t + k, what models/eagle3/metrics.py:16-119 does step by step.  Per-step quantities are [steps][T] by draft row.
+ *
+ * spx_loss_steps_mask: row_map [T] = rank of a target among the live ones (mask not zero) or -1, *live = their number; for
+ * step k, over its targets k, k + 1, ..: mask_sum[k] = the sum of the mask, full[k] = how many are live, inv[k] =
+ * step_weights[k] (host memory) / (mask_sum[k] + 1e-5); *ticket = 0 for spx_loss_steps_total.
+ *
+ * spx_loss_steps_pass: steps first .. end - 1 of `steps`, logits[k - first] (host array of device pointers) [T, vocab] with
+ * row stride ld_logits.  targets [T, vocab], or for ce NULL and argmax_target [T].  loss (0 where t + k >= T), tokens = the
+ * arg-max of every draft row, hits = it is the target's.  grad_logits (or NULL, with the four lists then): the row of
+ * step k at the live target of rank i is row i * steps + k, softmax(x) - softmax(y) (kl) or - onehot(argmax y) (ce);
+ * zeros where k exceeds the target's row.  row_slot [steps][T] = that row or -1, slot_row its inverse, *slots = live * steps,
+ * row_weight = mask * inv[k].  With grad_logits the losses of masked rows behind step 0 are written as 0.
+ *
+ * spx_loss_steps_total: out[k][8] as spx_ttt_step_total leaves it for every step, prev_correct (or NULL) [T] advanced over
+ * all steps, total = the sum of out[k][6].  partials: spx_loss_steps_partials floats. */
+#define SPX_LOSS_STEPS_MAX 32
+int spx_loss_steps_mask(const void* mask, int mask_kind, int64_t T, int32_t steps, const float* step_weights,
+                        int32_t* row_map, int32_t* live, float* inv, float* mask_sum, int32_t* full, int32_t* ticket,
+                        void* stream);
+int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld_logits, const void* targets, int64_t ld_targets,
+                        const int32_t* argmax_target, int64_t T, int64_t vocab, int32_t steps, int32_t first, int32_t end,
+                        const void* mask, int mask_kind, const float* inv, const int32_t* row_map, const int32_t* live,
+                        float* loss, int64_t* tokens, uint8_t* hits, int32_t* row_slot, int32_t* slot_row, int32_t* slots,
+                        float* row_weight, void* grad_logits, int64_t ld_grad, void* stream);
+int64_t spx_loss_steps_partials(int64_t T, int32_t steps);
+int spx_loss_steps_total(const float* loss, const uint8_t* hits, const void* mask, int mask_kind, void* prev_correct,
+                         int prev_kind, int64_t T, int32_t steps, float factor, const float* inv, const float* mask_sum,
+                         const int32_t* full, float* partials, int32_t* ticket, float* out, float* total, void* stream);
+
 /* Draft tokens: out[i] = known[i] for i < n (int32 arg-maxes of a loss pass, widened), out[n + j] = the first
  * index of the maximum of row j < tail of rows[tail, vocab] (bf16 / f32, row stride ld). */
 int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail, int64_t vocab,

@@ -48,6 +48,11 @@ SIGNATURES["spx_dflash_inputs_checked"] = [*SIGNATURES["spx_dflash_inputs"], _P]
 SIGNATURES["spx_ttt_step_terms"] = [_I32, _P, _P, _P, _I, _I64, _F, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_map"] = [_P, _I, _I64, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_lists"] = [_P, _I, _I64, _P, _P, _P, _P, _P]
+SIGNATURES["spx_loss_steps_mask"] = [_P, _I, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _P]
+SIGNATURES["spx_loss_steps_pass"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I32, _I32, _I32, _P, _I, _P, _P, _P, _P, _P, _P,
+                                     _P, _P, _P, _P, _P, _I64, _P]
+SIGNATURES["spx_loss_steps_partials"] = [_I64, _I32]
+SIGNATURES["spx_loss_steps_total"] = [_P, _P, _P, _I, _P, _I, _I64, _I32, _F, _P, _P, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_row_tokens"] = [_P, _I64, _P, _I64, _I64, _I64, _I, _P, _P]
 SIGNATURES["spx_span_attn_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _F, _P, _P,
                                    _P, _I64, _P]

@@ -132,6 +132,9 @@ PyMethodDef g_methods[] = {
     SPX_HOST("product_tn", spx_layer_product_tn)
     SPX_HOST("loss_step", spx_layer_loss_step)
     SPX_HOST("loss_terms", spx_layer_loss_terms)
+    SPX_HOST("loss_steps_begin", spx_layer_loss_steps_begin)
+    SPX_HOST("loss_steps_pass", spx_layer_loss_steps_pass)
+    SPX_HOST("loss_steps_end", spx_layer_loss_steps_end)
     SPX_HOST("cat_bf16", spx_layer_cat_bf16)
     SPX_HOST("gain_sums", spx_layer_gain_sums)
     {"set_error", set_error, METH_O, "the exception class raised for a failed call"},

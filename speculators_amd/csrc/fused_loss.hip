@@ -8,6 +8,7 @@
 // pre-scaled by log2(e), statistics are converted back at the end.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "loss_common.h"
 #include "../../include/spx.h"
@@ -1255,6 +1256,353 @@ __global__ __launch_bounds__(1024) void mask_row_map_kernel(const void* __restri
   pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, rows, row_map, count, row_of);
 }
 
+// op over the 64 lanes, every lane gets the result: moves inside the sixteen lanes of a row, then swaps of rows, where a
+// shuffle would be a trip through LDS (six of them a value: kl, 4096 rows x 7 steps 748 -> 719 us)
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_all(T v, Op op) {
+  static_assert(sizeof(T) == 4, "one register");
+  auto moved = [](T x, auto ctrl) __attribute__((always_inline)) {
+    const int i = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v = op(v, moved(v, std::integral_constant<int, 0xb1>{}));   // quad_perm 1 0 3 2
+  v = op(v, moved(v, std::integral_constant<int, 0x4e>{}));   // quad_perm 2 3 0 1
+  v = op(v, moved(v, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+  v = op(v, moved(v, std::integral_constant<int, 0x140>{}));  // row_mirror
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = op(__builtin_bit_cast(T, (uint32_t)rows[0]), __builtin_bit_cast(T, (uint32_t)rows[1]));
+  u = __builtin_bit_cast(uint32_t, v);
+  const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return op(__builtin_bit_cast(T, (uint32_t)halves[0]), __builtin_bit_cast(T, (uint32_t)halves[1]));
+}
+
+// ---- all steps of a TTT loop at one target row -------------------------------------------------------
+// Draft row t of step k meets target row t + k: one workgroup takes target row r and its draft rows (k, r - k), k = 0, 1, ..
+// one after the other, the target row in registers throughout: it is read once instead of once a step, and while a
+// step's gradient leaves, the next step's row is requested into the registers that it frees, so that the arithmetic of one
+// row runs beside the traffic of its neighbour.  Where r < k there is no such draft row, and the workgroup takes row T - k + r
+// instead, one of the k last, which have no target: its arg-max is a draft token like any other.  So every
+// (step, row) is met once.
+//   loss, tokens, hits, row_of_map, row_weight: [steps][T], indexed by draft row; grad and row_slot by slot, K a live
+//   target: slot = rank of the target among the live ones * K + k (k > r: a row of zeros, of weight zero).
+// kl, 7 steps of 4096 rows of 32000, 70 % live: a pass a step 1002 us, so 719 (4.7 TB/s; 5.3 for ce: the exponentials of kl
+// take as long as its traffic).  5 steps of 1999 rows without gradient 320 -> 208.
+struct StepsArgs {
+  const uint16_t* logits[SPX_LOSS_STEPS_MAX];  // [T, vocab] each
+  int64_t ld;
+  const uint16_t* targets;  // null: argmax_target is known (ce)
+  int64_t ld_targets;
+  const int32_t* argmax_target;
+  int T, vocab, steps, k0, k1;  // this launch: steps k0 .. k1 - 1 of `steps`
+  const void* mask;
+  int mask_kind;
+  const float* inv;             // [steps]: weight of a step's masked mean over the sum of its mask
+  const int32_t* row_map;       // [T]: rank of a live target, -1
+  const int32_t* live;          // live targets
+  float* loss;
+  int64_t* tokens;
+  uint8_t* hits;
+  int32_t* row_slot;            // GRAD ...
+  int32_t* slot_row;
+  int32_t* slots;
+  float* row_weight;
+  uint16_t* grad;
+  int64_t ld_grad;
+};
+
+template <int OP, bool GRAD>
+__global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void loss_steps_kernel(StepsArgs a) {
+  const int r = blockIdx.x, tid = threadIdx.x, T = a.T;
+  const int nchunks = a.vocab >> 3;
+  const int rank = GRAD ? a.row_map[r] : -1;
+  const bool live = rank >= 0;
+  auto row_of = [&](int k) __attribute__((always_inline)) { return r >= k ? r - k : T - k + r; };
+  auto unpack = [](u32x4 raw, float (&v)[8]) __attribute__((always_inline)) {
+    v[0] = bf16_lo(raw.x); v[1] = bf16_hi(raw.x); v[2] = bf16_lo(raw.y); v[3] = bf16_hi(raw.y);
+    v[4] = bf16_lo(raw.z); v[5] = bf16_hi(raw.z); v[6] = bf16_lo(raw.w); v[7] = bf16_hi(raw.w);
+  };
+  u32x4 xr[kFgChunks], yr[kFgChunks];
+  const uint16_t* xrow = a.logits[a.k0] + (int64_t)row_of(a.k0) * a.ld;
+  const uint16_t* const yrow = a.targets ? a.targets + (int64_t)r * a.ld_targets : nullptr;
+  if (a.targets) {
+#pragma unroll
+    for (int j = 0; j < kFgChunks; ++j) {
+      const int c = tid + j * kFgThreads;
+      if (c < nchunks) yr[j] = ld16(yrow + ((int64_t)c << 3));
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kFgChunks; ++j) {
+    const int c = tid + j * kFgThreads;
+    if (c < nchunks) xr[j] = ld16(xrow + ((int64_t)c << 3));
+  }
+  struct Part { float m, z, a, b; int i; };
+  __shared__ Part part[2][kFgWaves];
+  int turn = 0;
+  // every thread's (maximum, first index of it, sum of 2^(x' - max x'), sum) -> the workgroup's
+  auto reduce = [&](float& best, int& at, float& z, float& sum, bool soft) __attribute__((always_inline)) {
+    const float wb = wave_all(best, [](float x, float y) { return fmaxf(x, y); });
+    const int i = wave_all(best == wb ? at : 0x7fffffff, [](int x, int y) { return min(x, y); });
+    const float m = fmaxf(wb * kLog2e, kNegBig);
+    if (soft) {
+      const auto add = [](float x, float y) { return x + y; };
+      z = wave_all(z * fast_exp2(fmaxf(best * kLog2e, kNegBig) - m), add);
+      sum = wave_all(sum, add);
+    }
+    if ((tid & 63) == 0) part[turn][tid >> 6] = Part{m, z, sum, wb, i};
+    __syncthreads();
+    Part s = part[turn][0];
+#pragma unroll
+    for (int w = 1; w < kFgWaves; ++w) {
+      const Part o = part[turn][w];
+      if (o.b > s.b || (o.b == s.b && o.i < s.i)) { s.b = o.b; s.i = o.i; }
+      if (soft) {
+        const float mm = fmaxf(s.m, o.m);
+        s.z = s.z * fast_exp2(s.m - mm) + o.z * fast_exp2(o.m - mm);
+        s.a += o.a;
+        s.m = mm;
+      }
+    }
+    turn ^= 1;
+    best = s.b; at = (uint32_t)s.i < (uint32_t)a.vocab ? s.i : 0; z = s.m + fast_log2(s.z); sum = s.a;
+  };
+  auto largest = [&](const float (&x)[8], int base, float& best, int& at) __attribute__((always_inline)) {
+    float cx = x[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
+    if (cx > best) {  // strict: an earlier chunk of this thread keeps a tie
+      int k = 7;
+#pragma unroll
+      for (int i = 6; i >= 0; --i) k = (x[i] == cx) ? i : k;
+      best = cx; at = base + k;
+    }
+    return cx;
+  };
+  // max and sum of exponentials of a chunk into a thread's
+  auto soften = [&](const float (&x)[8], float cx, float& m, float& z) __attribute__((always_inline)) {
+    const float cs = cx * kLog2e;
+    if (cs > m) {
+      z *= fast_exp2(m - cs);
+      m = cs;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -m));
+  };
+
+  float lt2 = 0.f;  // base-2 log-sum-exp of the target row
+  int label;
+  if (a.targets) {
+    float best = -INFINITY, m = kNegBig, z = 0.f, none = 0.f;
+    label = 0x7fffffff;
+#pragma unroll
+    for (int j = 0; j < kFgChunks; ++j) {
+      const int c = tid + j * kFgThreads;
+      if (c >= nchunks) continue;
+      float y[8];
+      unpack(yr[j], y);
+      const float cy = largest(y, c << 3, best, label);
+      if (OP != SPX_LOSS_CE) soften(y, cy, m, z);
+    }
+    reduce(best, label, z, none, OP != SPX_LOSS_CE);
+    lt2 = z;
+  } else {
+    label = a.argmax_target[r];
+    if ((uint32_t)label >= (uint32_t)a.vocab) label = 0;
+  }
+  if (GRAD && r == 0 && tid == 0 && a.k0 == 0) *a.slots = *a.live * a.steps;
+  const float mask = mask_value(a.mask, a.mask_kind, r);
+
+  for (int k = a.k0; k < a.k1; ++k) {
+    const bool tail = r < k;
+    const int t = row_of(k);
+    // (nothing of the target row but its packed chunks stays in registers from step to step)
+    asm volatile("" : "+v"(label));
+#pragma unroll
+    for (int j = 0; j < kFgChunks; ++j)
+      if (OP == SPX_LOSS_KL) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+    // (a masked row's loss enters no mean: behind the first step it is not formed where gradients are)
+    const bool soft = !tail && (!GRAD || live || k == 0);
+    const bool more = k + 1 < a.k1;
+    const uint16_t* const nrow = more ? a.logits[k + 1] + (int64_t)row_of(k + 1) * a.ld : nullptr;
+    const bool early = more && !(GRAD && live);  // the row is read once: its registers are free chunk by chunk
+    float best = -INFINITY, m = kNegBig, z = 0.f, sum = 0.f;
+    int at = 0x7fffffff;
+    float xt = 0.f;
+    if (OP == SPX_LOSS_CE && tid == 0) xt = load1(xrow + label);
+#pragma unroll
+    for (int j = 0; j < kFgChunks; ++j) {
+      const int c = tid + j * kFgThreads;
+      if (c >= nchunks) continue;
+      float x[8];
+      unpack(xr[j], x);
+      if (early) xr[j] = ld16(nrow + ((int64_t)c << 3));
+      const float cx = largest(x, c << 3, best, at);
+      if (soft) {
+        soften(x, cx, m, z);
+        if (OP == SPX_LOSS_KL) {
+          float y[8];
+          unpack(yr[j], y);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sum = fmaf(fast_exp2(fmaf(y[i], kLog2e, -lt2)), y[i] - x[i], sum);
+        }
+      }
+    }
+    reduce(best, at, z, sum, soft);
+    if (tid == 0) {
+      const int64_t g = (int64_t)k * T + t;
+      float row_loss = 0.f;
+      if (soft) row_loss = OP == SPX_LOSS_KL ? sum - lt2 * kLn2 + z * kLn2 : z * kLn2 - xt;
+      a.loss[g] = row_loss;
+      a.tokens[g] = at;
+      a.hits[g] = at == label;
+      if (GRAD) {
+        const int slot = live ? rank * a.steps + k : -1;
+        a.row_slot[g] = tail ? -1 : slot;
+        if (live) a.slot_row[slot] = (int)g;
+        a.row_weight[g] = tail ? 0.f : mask * a.inv[k];
+      }
+    }
+    if (GRAD && live) {
+      uint16_t* const grow = a.grad + ((int64_t)rank * a.steps + k) * a.ld_grad;
+      const float cd = -z, ct = -lt2;
+#pragma unroll
+      for (int j = 0; j < kFgChunks; ++j) {  // (the packed chunks are what stays in registers between the passes)
+        asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
+        if (OP == SPX_LOSS_KL) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+      }
+#pragma unroll
+      for (int j = 0; j < kFgChunks; ++j) {
+        const int c = tid + j * kFgThreads;
+        if (c >= nchunks) continue;
+        const int base = c << 3;
+        float x[8], y[8], o[8];
+        unpack(xr[j], x);
+        if (OP == SPX_LOSS_KL) unpack(yr[j], y);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float dp = fast_exp2(fmaf(x[i], kLog2e, cd));
+          if (OP == SPX_LOSS_CE) o[i] = dp - ((base + i) == label ? 1.f : 0.f);
+          else o[i] = dp - fast_exp2(fmaf(y[i], kLog2e, ct));
+          if (tail) o[i] = 0.f;
+        }
+        store8_vec<uint16_t>(grow + base, o);
+        if (more) xr[j] = ld16(nrow + base);
+      }
+    }
+    xrow = nrow;
+  }
+}
+
+// What the passes of loss_steps_kernel need of the mask: the live targets in order, and for every step the weight of its
+// mean over the sum of the mask of its targets (k, k + 1, ..), how many of them are live, and that sum.  One workgroup.
+struct StepWeights { float w[SPX_LOSS_STEPS_MAX]; };
+__global__ __launch_bounds__(1024) void steps_mask_kernel(const void* __restrict__ mask, int mask_kind, int T, int steps,
+                                                          StepWeights weights, int32_t* __restrict__ row_map,
+                                                          int32_t* __restrict__ live, float* __restrict__ inv,
+                                                          float* __restrict__ msum, int32_t* __restrict__ full,
+                                                          int32_t* __restrict__ ticket) {
+  __shared__ float fl[16];
+  __shared__ int il[16];
+  pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, T, row_map, live);
+  float s = 0.f;
+  int n = 0;
+  for (int r = steps - 1 + threadIdx.x; r < T; r += 1024) {  // (steps <= T)
+    const float v = mask_value(mask, mask_kind, r);
+    s += v;
+    n += v != 0.f;
+  }
+  s = block_sum_f(s, fl);
+  n = block_sum_i(n, il);
+  if (threadIdx.x == 0) {
+    *ticket = 0;
+    for (int k = steps - 1; k >= 0; --k) {
+      if (k < steps - 1) {
+        const float v = mask_value(mask, mask_kind, k);
+        s += v;
+        n += v != 0.f;
+      }
+      msum[k] = s;
+      full[k] = n;
+      inv[k] = weights.w[k] / (s + 1e-5f);
+    }
+  }
+}
+
+// Behind the row passes: the acceptance chain along a draft row's steps, every step's masked mean and counts (as
+// ttt_step_reduce_kernel leaves them in out[k][8]) and the loss.  A thread owns a draft row; the workgroups' partial sums are
+// added in their order by the one that arrives last, which resets nothing and waits for nothing.
+constexpr int kStepsRows = 256;
+__global__ __launch_bounds__(kStepsRows) void steps_total_kernel(
+    const float* __restrict__ loss, const uint8_t* __restrict__ hits, const void* __restrict__ mask, int mask_kind,
+    void* prev, int prev_kind, int T, int steps, float factor, const float* __restrict__ inv, const float* __restrict__ msum,
+    const int32_t* __restrict__ full, float* __restrict__ partial, int32_t* __restrict__ ticket, float* __restrict__ out,
+    float* __restrict__ total) {
+  __shared__ float ls[kStepsRows / 64][SPX_LOSS_STEPS_MAX];
+  __shared__ int cs[kStepsRows / 64][SPX_LOSS_STEPS_MAX][2];
+  __shared__ int last;
+  __shared__ float parts[SPX_LOSS_STEPS_MAX];
+  const int t = blockIdx.x * kStepsRows + threadIdx.x, wave = threadIdx.x >> 6;
+  bool was = t < T && (!prev || mask_value(prev, prev_kind, t) != 0.f);
+  for (int k = 0; k < steps; ++k) {
+    float l = 0.f;
+    bool good = false, chained = false;
+    if (t < T - k) {
+      const float m = mask_value(mask, mask_kind, t + k);
+      l = fmaf(loss[(int64_t)k * T + t], m, 0.f);
+      chained = was;
+      was = was && hits[(int64_t)k * T + t];
+      good = was && m != 0.f;
+    }
+    l = wave_sum(l);
+    const int correct = __popcll(__ballot(good)), cond = __popcll(__ballot(chained));
+    if ((threadIdx.x & 63) == 0) { ls[wave][k] = l; cs[wave][k][0] = correct; cs[wave][k][1] = cond; }
+  }
+  if (prev && t < T) store_flag(prev, prev_kind, t, was);
+  __syncthreads();
+  if ((int)threadIdx.x < steps) {
+    const int k = threadIdx.x;
+    float l = 0.f;
+    int c = 0, d = 0;
+    for (int w = 0; w < kStepsRows / 64; ++w) { l += ls[w][k]; c += cs[w][k][0]; d += cs[w][k][1]; }
+    float* const p = partial + ((int64_t)blockIdx.x * steps + k) * 3;
+    __hip_atomic_store(p, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, __int_as_float(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 2, __int_as_float(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  if ((int)threadIdx.x < steps) {
+    const int k = threadIdx.x;
+    float l = 0.f;
+    int c = 0, d = 0;
+    for (int b = 0; b < (int)gridDim.x; ++b) {
+      const float* const p = partial + ((int64_t)b * steps + k) * 3;
+      l += __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      c += __float_as_int(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      d += __float_as_int(__hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    float* const o = out + 8 * k;
+    o[0] = l * inv[k];
+    o[1] = o[3] = (float)c;
+    o[2] = (float)full[k];
+    o[4] = (float)d;
+    o[5] = msum[k];
+    o[6] = parts[k] = l * inv[k] * factor;
+    o[7] = 1.f;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float sum = parts[0];
+    for (int k = 1; k < steps; ++k) sum += parts[k];
+    *total = sum;
+  }
+}
+
 // Draft tokens (int64): the known arg-maxes of the first n rows widened, the arg-max (first index of the
 // maximum) of the rows behind them, one workgroup each.  One launch for a conversion, an arg-max pass over few
 // rows, another conversion and a concatenation.  A handful of rows is a chain of loads: with 1024 threads to a row
@@ -1786,6 +2134,83 @@ extern "C" int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows,
 extern "C" int spx_mask_row_map(const void* mask, int mask_kind, int64_t rows, int32_t* row_map, int32_t* count,
                                 int32_t* zero3, void* stream) {
   return spx_mask_row_lists(mask, mask_kind, rows, row_map, count, nullptr, zero3, stream);
+}
+
+static bool steps_ok(int64_t T, int32_t steps) {
+  return steps > 0 && steps <= SPX_LOSS_STEPS_MAX && T >= steps && T * steps < (1ll << 31);
+}
+
+extern "C" int spx_loss_steps_mask(const void* mask, int mask_kind, int64_t T, int32_t steps, const float* step_weights,
+                                   int32_t* row_map, int32_t* live, float* inv, float* mask_sum, int32_t* full,
+                                   int32_t* ticket, void* stream) {
+  SPX_REQUIRE(steps_ok(T, steps), "1 .. 32 steps, no more than rows");
+  SPX_REQUIRE(mask && step_weights && row_map && live && inv && mask_sum && full && ticket, "null buffer");
+  SPX_REQUIRE(kind_ok(mask_kind), "unknown mask element kind");
+  StepWeights w{};
+  for (int k = 0; k < steps; ++k) w.w[k] = step_weights[k];
+  hipLaunchKernelGGL(steps_mask_kernel, dim3(1), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), mask, mask_kind,
+                     (int)T, steps, w, row_map, live, inv, mask_sum, full, ticket);
+  return check_launch(__func__);
+}
+
+extern "C" int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld_logits, const void* targets,
+                                   int64_t ld_targets, const int32_t* argmax_target, int64_t T, int64_t vocab,
+                                   int32_t steps, int32_t first, int32_t end, const void* mask, int mask_kind,
+                                   const float* inv, const int32_t* row_map, const int32_t* live, float* loss,
+                                   int64_t* tokens, uint8_t* hits, int32_t* row_slot, int32_t* slot_row, int32_t* slots,
+                                   float* row_weight, void* grad_logits, int64_t ld_grad, void* stream) {
+  SPX_REQUIRE(op == SPX_LOSS_KL || op == SPX_LOSS_CE, "built for kl and ce");
+  SPX_REQUIRE(steps_ok(T, steps) && first >= 0 && first < end && end <= steps, "1 .. 32 steps, no more than rows");
+  SPX_REQUIRE(vocab > 0 && vocab % 8 == 0 && vocab <= (int64_t)kFgThreads * kFgChunks * 8,
+              "vocab must be a multiple of 8, at most 32768");
+  SPX_REQUIRE(targets || (op == SPX_LOSS_CE && argmax_target), "no targets");
+  SPX_REQUIRE(ld_logits >= vocab && ld_logits % 8 == 0 && (!targets || (ld_targets >= vocab && ld_targets % 8 == 0)) &&
+                  (!grad_logits || (ld_grad >= vocab && ld_grad % 8 == 0)),
+              "row strides must be multiples of 8 elements, at least vocab");
+  SPX_REQUIRE(logits && mask && inv && loss && tokens && hits, "null buffer");
+  SPX_REQUIRE(kind_ok(mask_kind), "unknown mask element kind");
+  SPX_REQUIRE(!grad_logits || (row_map && live && row_slot && slot_row && slots && row_weight), "null buffer");
+  SPX_REQUIRE((!targets || aligned16(targets)) && (!grad_logits || aligned16(grad_logits)), "rows must be 16-byte aligned");
+  StepsArgs a{};
+  for (int k = first; k < end; ++k) {
+    SPX_REQUIRE(logits[k - first] && aligned16(logits[k - first]), "null or unaligned logits");
+    a.logits[k] = reinterpret_cast<const uint16_t*>(logits[k - first]);
+  }
+  a.ld = ld_logits;
+  a.targets = reinterpret_cast<const uint16_t*>(targets);
+  a.ld_targets = ld_targets;
+  a.argmax_target = argmax_target;
+  a.T = (int)T; a.vocab = (int)vocab; a.steps = steps; a.k0 = first; a.k1 = end;
+  a.mask = mask; a.mask_kind = mask_kind; a.inv = inv;
+  a.row_map = row_map; a.live = live;
+  a.loss = loss; a.tokens = tokens; a.hits = hits;
+  a.row_slot = row_slot; a.slot_row = slot_row; a.slots = slots; a.row_weight = row_weight;
+  a.grad = reinterpret_cast<uint16_t*>(grad_logits);
+  a.ld_grad = ld_grad;
+  const dim3 grid((unsigned)T), block(kFgThreads);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+#define SPX_SP(OPV, G) hipLaunchKernelGGL((loss_steps_kernel<OPV, G>), grid, block, 0, st, a)
+  if (op == SPX_LOSS_KL) { if (grad_logits) SPX_SP(SPX_LOSS_KL, true); else SPX_SP(SPX_LOSS_KL, false); }
+  else { if (grad_logits) SPX_SP(SPX_LOSS_CE, true); else SPX_SP(SPX_LOSS_CE, false); }
+#undef SPX_SP
+  return check_launch(__func__);
+}
+
+extern "C" int64_t spx_loss_steps_partials(int64_t T, int32_t steps) {
+  return T <= 0 || steps <= 0 ? 0 : (T + kStepsRows - 1) / kStepsRows * steps * 3;
+}
+
+extern "C" int spx_loss_steps_total(const float* loss, const uint8_t* hits, const void* mask, int mask_kind,
+                                    void* prev_correct, int prev_kind, int64_t T, int32_t steps, float factor,
+                                    const float* inv, const float* mask_sum, const int32_t* full, float* partials,
+                                    int32_t* ticket, float* out, float* total, void* stream) {
+  SPX_REQUIRE(steps_ok(T, steps), "1 .. 32 steps, no more than rows");
+  SPX_REQUIRE(loss && hits && mask && inv && mask_sum && full && partials && ticket && out && total, "null buffer");
+  SPX_REQUIRE(kind_ok(mask_kind) && (!prev_correct || kind_ok(prev_kind)), "unknown element kind");
+  hipLaunchKernelGGL(steps_total_kernel, dim3((unsigned)((T + kStepsRows - 1) / kStepsRows)), dim3(kStepsRows), 0,
+                     reinterpret_cast<hipStream_t>(stream), loss, hits, mask, mask_kind, prev_correct, prev_kind, (int)T,
+                     steps, factor, inv, mask_sum, full, partials, ticket, out, total);
+  return check_launch(__func__);
 }
 
 extern "C" int spx_row_tokens(const int32_t* known, int64_t n, const void* rows, int64_t ld, int64_t tail,

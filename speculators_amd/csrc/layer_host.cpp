@@ -450,6 +450,120 @@ PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The loss of all steps of a TTT loop (spx_loss_steps_*).  What its launches share lies in two buffers:
+struct LossSteps {
+  int64_t T, steps;
+  int32_t *row_map, *live, *slots, *ticket, *full, *row_slot, *slot_row;
+  float *inv, *mask_sum, *loss, *row_weight, *partials;
+  static int64_t ints(int64_t T, int64_t steps) { return T + 3 + steps + 2 * steps * T; }
+  static int64_t floats_of(int64_t T, int64_t steps) { return 2 * steps + 2 * steps * T + spx_loss_steps_partials(T, (int32_t)steps); }
+  LossSteps(const Tensor& i, const Tensor& f, int64_t T_, int64_t steps_) : T(T_), steps(steps_) {
+    TORCH_CHECK_VALUE(i.scalar_type() == at::kInt && f.scalar_type() == at::kFloat && i.is_contiguous() && f.is_contiguous() &&
+                          i.numel() == ints(T, steps) && f.numel() == floats_of(T, steps),
+                      "the buffers of loss_steps_begin for ", T, " rows and ", steps, " steps");
+    row_map = i.mutable_data_ptr<int32_t>();
+    live = row_map + T; slots = live + 1; ticket = slots + 1; full = ticket + 1; row_slot = full + steps;
+    slot_row = row_slot + steps * T;
+    inv = f.mutable_data_ptr<float>();
+    mask_sum = inv + steps; loss = mask_sum + steps; row_weight = loss + steps * T; partials = row_weight + steps * T;
+  }
+};
+
+// (mask, its kind, the steps' weights ..) -> (integers, floats; views: live slots, row -> slot, slot -> row, row weights)
+PyObject* spx_layer_loss_steps_begin(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const int64_t steps = n - 2;
+  TORCH_CHECK_TYPE(steps >= 1 && steps <= SPX_LOSS_STEPS_MAX, "loss_steps_begin takes 1 .. 32 step weights");
+  Args x("loss_steps_begin", args, n, n);
+  const Tensor& mask = x.tensor();
+  const int64_t kind = x.integer();
+  float weights[SPX_LOSS_STEPS_MAX];
+  for (int64_t k = 0; k < steps; ++k) weights[k] = (float)x.number();
+  Unlocked released;
+  const int64_t T = mask.numel();
+  const Tensor i = at::empty({LossSteps::ints(T, steps)}, mask.options().dtype(at::kInt).requires_grad(false)),
+               f = at::empty({LossSteps::floats_of(T, steps)}, mask.options().dtype(at::kFloat).requires_grad(false));
+  const LossSteps s(i, f, T, steps);
+  check(spx_loss_steps_mask(mask.const_data_ptr(), kind, T, (int32_t)steps, weights, s.row_map, s.live, s.inv, s.mask_sum,
+                            s.full, s.ticket, stream_of(mask)),
+        "spx_loss_steps_mask");
+  const int64_t lists = s.row_slot - s.row_map, w = s.row_weight - s.inv;
+  return tuple_of(released, {i, f, i.narrow(0, T + 1, 1), i.narrow(0, lists, steps * T),
+                             i.narrow(0, lists + steps * T, steps * T), f.narrow(0, w, steps * T)});
+  END_HANDLE_TH_ERRORS
+}
+
+// (op, mask, its kind, targets or None, their arg-max or None, integers, floats, tokens [steps, T], hits [steps, T], packed
+// gradient [steps * T, vocab] or None, steps, first step, logits [T, vocab] of this and the following steps ..)
+PyObject* spx_layer_loss_steps_pass(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const int64_t here = n - 12;
+  TORCH_CHECK_TYPE(here >= 1 && here <= SPX_LOSS_STEPS_MAX, "loss_steps_pass takes the logits of 1 .. 32 steps");
+  Args x("loss_steps_pass", args, n, n);
+  const int64_t op = x.integer();
+  const Tensor& mask = x.tensor();
+  const int64_t kind = x.integer();
+  const Tensor y = x.maybe(), known = x.maybe();
+  const Tensor &i = x.tensor(), &f = x.tensor(), &tokens = x.tensor(), &hits = x.tensor();
+  const Tensor packed = x.maybe();
+  const int64_t steps = x.integer(), first = x.integer();
+  const void* logits[SPX_LOSS_STEPS_MAX];
+  int64_t vocab = 0, ld = 0;
+  const int64_t T = mask.numel();
+  for (int64_t k = 0; k < here; ++k) {
+    const Tensor& l = x.tensor();
+    if (k == 0) { vocab = l.size(1); ld = l.stride(0); }
+    TORCH_CHECK_VALUE(l.dim() == 2 && l.size(0) == T && l.size(1) == vocab && l.stride(0) == ld && l.stride(1) == 1 &&
+                          l.scalar_type() == at::kBFloat16 && l.device() == mask.device(),
+                      "bf16 logits [rows, vocab], all alike");
+    logits[k] = l.const_data_ptr();
+  }
+  TORCH_CHECK_VALUE((!y.defined() || (y.size(0) == T && y.size(1) == vocab && y.stride(1) == 1 && y.scalar_type() == at::kBFloat16)) &&
+                        (!known.defined() || (known.numel() == T && known.is_contiguous() && known.scalar_type() == at::kInt)) &&
+                        tokens.numel() == steps * T && hits.numel() == steps * T && tokens.scalar_type() == at::kLong &&
+                        hits.scalar_type() == at::kByte && tokens.is_contiguous() && hits.is_contiguous() &&
+                        (!packed.defined() || (packed.numel() == steps * T * vocab && packed.is_contiguous() &&
+                                               packed.scalar_type() == at::kBFloat16)),
+                    "targets, their arg-max, tokens, hits or gradient do not fit the logits");
+  Unlocked released;
+  const LossSteps s(i, f, T, steps);
+  check(spx_loss_steps_pass((int)op, logits, ld, y.defined() ? in(y) : nullptr, y.defined() ? y.stride(0) : 0,
+                            known.defined() ? known.const_data_ptr<int32_t>() : nullptr, T, vocab, (int32_t)steps,
+                            (int32_t)first, (int32_t)(first + here), mask.const_data_ptr(), kind, s.inv, s.row_map, s.live,
+                            s.loss, tokens.mutable_data_ptr<int64_t>(), hits.mutable_data_ptr<uint8_t>(), s.row_slot,
+                            s.slot_row, s.slots, s.row_weight, packed.defined() ? to(packed) : nullptr, vocab,
+                            stream_of(mask)),
+        "spx_loss_steps_pass");
+  released.lock();
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// (mask, its kind, prev or None, its kind, integers, floats, hits, steps, term factor) -> (scalars [steps, 8], loss)
+PyObject* spx_layer_loss_steps_end(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args x("loss_steps_end", args, n, 9);
+  const Tensor& mask = x.tensor();
+  const int64_t kind = x.integer();
+  const Tensor prev = x.maybe();
+  const int64_t prev_kind = x.integer();
+  const Tensor &i = x.tensor(), &f = x.tensor(), &hits = x.tensor();
+  const int64_t steps = x.integer();
+  const double factor = x.number();
+  const int64_t T = mask.numel();
+  TORCH_CHECK_VALUE(hits.numel() == steps * T && (!prev.defined() || (prev.numel() >= T && prev.is_contiguous())),
+                    "hits or prev do not fit the mask");
+  Unlocked released;
+  const LossSteps s(i, f, T, steps);
+  const Tensor out = at::empty({steps, 8}, f.options()), total = at::empty({}, f.options());
+  check(spx_loss_steps_total(s.loss, hits.const_data_ptr<uint8_t>(), mask.const_data_ptr(), kind,
+                             prev.defined() ? prev.mutable_data_ptr() : nullptr, prev_kind, T, (int32_t)steps, (float)factor,
+                             s.inv, s.mask_sum, s.full, s.partials, s.ticket, floats(out), floats(total), stream_of(mask)),
+        "spx_loss_steps_total");
+  return tuple_of(released, {out, total});
+  END_HANDLE_TH_ERRORS
+}
+
 // The row-wise concatenation of one to four matrices as one bf16 matrix
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS

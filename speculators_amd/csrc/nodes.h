@@ -19,5 +19,8 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
 PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_loss_steps_begin(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_loss_steps_pass(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_loss_steps_end(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_gain_sums(PyObject*, PyObject* const* args, Py_ssize_t n);

@@ -396,6 +396,7 @@ class Eagle3DraftModel(nn.Module):
         rope_top = self._rotary.top(position_ids)
         draft_tokens = []
         self.last_logits = []
+        together = None
         for step in range(ttt_steps):
             # looked up once for all steps (a step's rows are a window of them), without a graph whatever
             # embed_requires_grad says, as the reference does (models/eagle3/core.py:270-271): the flag only marks
@@ -423,8 +424,17 @@ class Eagle3DraftModel(nn.Module):
                     y = _Prenormed(y, normed)
             hidden = normed if cfg.norm_output else y
             head = self._stager.get(self.lm_head.weight)
-            fuse = (return_loss and self.fuse_head_loss and normed.requires_grad
-                    and not head.trainable)
+            frozen = return_loss and self.fuse_head_loss and not head.trainable
+            fuse = frozen and normed.requires_grad
+            if step == 0 and frozen:
+                # head and loss of all steps behind the last of them (see metrics.TTTSteps)
+                together = MT.TTTSteps.take(normed, head.w, targets, loss_mask, prev_correct, ttt_steps, ttt_step_loss_decay,
+                                            loss_config)
+            if together is not None:
+                together.add(normed)
+                full_mask = None if full_mask is None else full_mask.extended()
+                sw_mask = None if sw_mask is None else sw_mask.extended()
+                continue
             if not fuse:
                 logits = gemm.linear_staged(normed, head, hip=True)
 
@@ -452,6 +462,9 @@ class Eagle3DraftModel(nn.Module):
 
         if not return_loss:
             return draft_tokens
+        if together is not None:
+            loss, metrics, draft_tokens = together.finish(head.w, head.wt if normed.requires_grad else None,
+                                                          self.last_logits if self.keep_logits else None)
         if loss is None:
             loss = torch.zeros((), device=device)
         metrics["loss_sum"] = loss.detach().clone()

@@ -510,6 +510,93 @@ def head_terms_loss(loss_config, x, weight, weight_t, targets, d2t, target_stats
     return total, am_d, am_t, lse_t, logits.view(1, t, weight.shape[0])
 
 
+LOSS_STEPS_MAX = 32            # SPX_LOSS_STEPS_MAX
+STEPS_LOGITS_BYTES = 1 << 32   # logits of several steps that are held at a time (at least one step's)
+
+
+class _HeadStepsLoss(torch.autograd.Function):
+    """``_HeadStepLoss`` of all steps of a TTT loop at once: ``(x of every step) -> total``.  A target row meets the draft
+    rows of all steps in one workgroup (``spx_loss_steps_pass``), and the backward is ONE input-gradient product over the live
+    rows of all steps.  Everything else comes back in ``run``."""
+
+    @staticmethod
+    def forward(ctx, run, weight, weight_t, *xs):
+        from .gemm import matmul_nt
+
+        t, vocab, steps = run.mask.numel(), weight.shape[0], len(xs)
+        dev = weight.device
+        native = _lib.native()
+        kind = _lib.kind_code(run.mask)
+        grad = run.grad
+        ints, floats, count, row_slot, slot_row, row_weight = native.loss_steps_begin(run.mask, kind, *run.weights)
+        run.tokens = torch.empty(steps, t, device=dev, dtype=torch.int64)
+        hits = torch.empty(steps, t, device=dev, dtype=torch.uint8)
+        packed = torch.empty(steps * t, vocab, device=dev, dtype=torch.bfloat16) if grad else None
+        at_once = max(1, STEPS_LOGITS_BYTES // (2 * t * vocab))
+        for first in range(0, steps, at_once):
+            logits = [matmul_nt(x.reshape(t, x.shape[-1]), weight) for x in xs[first:first + at_once]]
+            native.loss_steps_pass(run.op, run.mask, kind, run.targets, run.argmax, ints, floats, run.tokens, hits, packed, steps,
+                                   first, *logits)
+            if run.logits is not None:
+                run.logits += logits
+        run.scalars, total = native.loss_steps_end(
+            run.mask, kind, run.prev, _lib.kind_code(run.prev) if run.prev is not None else 0, ints, floats, hits, steps,
+            run.factor)
+        if grad:
+            ctx.save_for_backward(packed, row_slot, count, weight_t, row_weight, slot_row)
+        ctx.factor, ctx.shapes = run.factor, [x.shape for x in xs]
+        return total
+
+    @staticmethod
+    def backward(ctx, g):
+        steps = len(ctx.shapes)
+        row_slot = ctx.saved_tensors[1]
+        dx = _unit_rows_backward(ctx.saved_tensors, g.to(torch.float32), ctx.factor, row_slot.numel())
+        return (None, None, None) + tuple(d.view(shape) for d, shape in zip(dx.chunk(steps), ctx.shapes, strict=True))
+
+
+@dataclass
+class HeadSteps:
+    """One loss (``op``: kl or ce) of all steps behind the frozen head: per-step ``weights`` of the masked mean, the term's
+    ``factor``, 1-D ``mask`` and ``prev`` (advanced in place), ``targets`` ``[T, vocab]`` or for ce their ``argmax``.  Filled
+    by ``head_steps_loss``: ``tokens`` int64 ``[steps, T]``, ``scalars`` f32 ``[steps, 8]`` (``spx_ttt_step_total``) and,
+    where it is a list before, ``logits``."""
+
+    op: int
+    weights: list
+    factor: float
+    mask: torch.Tensor
+    prev: torch.Tensor | None
+    targets: torch.Tensor | None
+    argmax: torch.Tensor | None
+    logits: list | None = None
+    grad: bool = False
+    tokens: torch.Tensor | None = None
+    scalars: torch.Tensor | None = None
+
+
+def steps_fit(op: int, steps: int, x, weight, targets, mask) -> bool:
+    """Whether ``head_steps_loss`` takes the steps: rows of the targets (``[T, vocab]``; None: ce by known arg-max) and
+    logits that fit a workgroup's registers, as ``_one_pass_ok``, of 4096 columns on as ``TERMS_MIN_VOCAB``.  From two
+    steps on: it has something to share."""
+    if not (HEAD_LOSS_ONE_PASS and 2 <= steps <= LOSS_STEPS_MAX and op in (OP_KL, OP_CE) and mask is not None):
+        return False
+    t, vocab = mask.numel(), weight.shape[0]
+    if (t < steps or t * steps >= 1 << 31 or x.shape[:-1] != (1, t) or x.dtype != torch.bfloat16
+            or weight.dtype != torch.bfloat16 or vocab % 8 or not TERMS_MIN_VOCAB <= vocab <= 32768):
+        return False
+    if targets is None:
+        return op == OP_CE
+    return (targets.dtype == torch.bfloat16 and targets.shape == (t, vocab) and targets.stride(1) == 1
+            and targets.stride(0) % 8 == 0 and targets.data_ptr() % 16 == 0)
+
+
+def head_steps_loss(run: HeadSteps, weight, weight_t, xs):
+    """The loss of all steps (``steps_fit``) over ``xs``, every step's ``[1, T, H]``, behind the frozen head ``weight``."""
+    run.grad = torch.is_grad_enabled() and any(x.requires_grad for x in xs)
+    return _HeadStepsLoss.apply(run, weight, weight_t, *xs)
+
+
 def _check_head(x, weight, targets, n: int):
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise _lib.SpxError("head_fused_rows takes bf16 operands")

@@ -180,6 +180,73 @@ def _terms_step(head, targets, loss_mask, prev_correct, ttt_step, decay, loss_co
     return (total, m, am_d) if return_pred else (total, m)
 
 
+def _steps_targets(targets, op: int):
+    """``(rows [T, vocab], arg-max)`` of the verifier for ``losses.head_steps_loss``: for ce behind the lazily applied head
+    the arg-max alone."""
+    if isinstance(targets, VerifierHead):
+        if op == L.OP_CE and targets.logits is None:
+            return None, targets.stats()[1]
+        targets = targets.materialize()
+    return targets[0], None
+
+
+class TTTSteps:
+    """``compute_metrics`` of all steps of a TTT loop at once, where one node takes them (``losses.head_steps_loss``):
+    a loss of one kl or ce term over bf16 rows, with a loss mask.  ``add`` a step's head input, ``finish`` behind the last."""
+
+    def __init__(self, op, steps, targets, loss_mask, prev_correct, decay, factor):
+        self.op, self.steps, self.targets = op, steps, targets
+        self.mask, self.prev, self.factor = loss_mask, prev_correct, factor
+        self.weights = [float(np.float32(decay) ** np.float32(k)) for k in range(steps)]
+        self.xs = []
+
+    @staticmethod
+    def take(x, weight, targets, loss_mask, prev_correct, steps, decay, loss_config):
+        """The steps behind ``x`` (the first one's head input), or None where ``compute_metrics`` has to take them."""
+        if loss_config is None:
+            loss_config = {"kl_div": (L.kl_div_loss, 1.0)}
+        if (compute_metrics is not _own_compute_metrics or len(loss_config) != 1 or loss_mask is None
+                or isinstance(targets, TargetGather)):
+            return None
+        (name, (fn, factor)), = loss_config.items()
+        op = L.PRIMITIVE_OP.get(name)
+        if op not in (L.OP_KL, L.OP_CE) or fn is not L._HIP_LOSS_FN_MAP[name]:
+            return None
+        shape = tuple(x.shape[:-1])
+        if shape[0] != 1 or tuple(loss_mask.shape) != shape or tuple(prev_correct.shape) != shape:
+            return None
+        rows = None
+        if isinstance(targets, VerifierHead):  # (its rows are bf16, contiguous, of its weight's width)
+            fits = targets.x.shape[1] == shape[1] and targets.weight.shape[0] == weight.shape[0]
+            op_rows = L.steps_fit(L.OP_CE, steps, x, weight, None, loss_mask)
+            if not (fits and op_rows and targets.weight.dtype == torch.bfloat16):
+                return None
+        else:
+            rows = targets[0] if targets.dim() == 3 and targets.shape[0] == 1 else None
+            if rows is None or not L.steps_fit(op, steps, x, weight, rows, loss_mask):
+                return None
+        return TTTSteps(op, steps, targets, _as_mask(loss_mask), _flat_prev(prev_correct), decay, float(factor))
+
+    def add(self, x):
+        self.xs.append(x)
+
+    def finish(self, weight, weight_t, logits=None):
+        """``(loss, metrics, draft tokens of every step [1, T])``; ``logits``: a list that receives every step's."""
+        rows, argmax = _steps_targets(self.targets, self.op)
+        kept = None if logits is None else []
+        run = L.HeadSteps(self.op, self.weights, self.factor, self.mask, self.prev, rows, argmax, kept)
+        loss = L.head_steps_loss(run, weight, weight_t, self.xs)
+        if logits is not None:
+            logits += [x.view(1, *x.shape) for x in kept]
+        m = {}
+        for k in range(self.steps):
+            out = run.scalars[k]
+            m[f"loss_{k}_sum"], m[f"loss_{k}_total"] = out[6], out[7]
+            m[f"full_acc_{k}_sum"], m[f"full_acc_{k}_total"] = out[1], out[2]
+            m[f"cond_acc_{k}_sum"], m[f"cond_acc_{k}_total"] = out[3], out[4]
+        return loss, m, list(run.tokens.split(1))
+
+
 def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
                     ttt_step_loss_decay: float, loss_config: L.LossConfig | None = None,
                     target_stats_cache: dict | None = None, return_pred: bool = False,
@@ -321,6 +388,9 @@ def compute_metrics(logits, targets, loss_mask, prev_correct, ttt_step: int,
     if return_pred:
         return total, m, pred
     return total, m
+
+
+_own_compute_metrics = compute_metrics  # (a replaced one is called, step by step)
 
 
 def row_tokens(known, rows: torch.Tensor) -> torch.Tensor:
