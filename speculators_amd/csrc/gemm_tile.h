@@ -184,6 +184,26 @@ struct Operand {
   }
 };
 
+// us of the pass that adds the parts of `partials` fp32 results in all
+__host__ __device__ __forceinline__ float reduce_us(float partials) { return 4.1f + 1.03e-6f * partials; }
+
+// The parts of a product whose rows are counted on the device: those that make it shortest, as the host has it for all M rows
+// (choose in gemm_tile.hip), for the tiles that are there.  max_parts = 0: as the host says.
+struct LiveCut {
+  int max_parts, cap, slabs;  // cap: workgroups the chip holds
+  float s0, s1;               // of the tile's Config
+  __device__ __forceinline__ int parts(int tiles, float results) const {
+    int best = 1;
+    float us = 3.4e38f;
+    for (int n = 1; n <= max_parts && (n == 1 || tiles * n <= cap); ++n) {
+      const float t = (s0 + s1 * (float)min(tiles * n, cap) / (float)cap) * (float)((slabs + n - 1) / n) +
+                      (n > 1 ? reduce_us((float)n * results) : 0.f);
+      if (t < us) { us = t; best = n; }
+    }
+    return tiles > 0 ? best : 1;
+  }
+};
+
 struct Params {
   const uint16_t* A;
   const uint16_t* B;
@@ -200,6 +220,7 @@ struct Params {
   const int32_t* src;           // PICK: where each of the operand's rows lies in the matrix it is picked from ...
   int src_rows;                 // ... and that matrix's rows
   RowGrade grade;               // GRADE: what the rows are multiplied by
+  LiveCut cut;                  // GRADE: parts by the rows that count, [parts][whole tile rows of them][N] then
 };
 
 // OUT: 0 = bf16, 1 = bf16 added to C, 2 = fp32, 3 = fp32 added to C.  STREAM: non-temporal stores (OUT 0 and 2).  GRADE: rows
@@ -228,7 +249,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
     tiles_m = (M + TM - 1) / TM;
   }
   if (!AT && p.tile_tab) tiles_m = min(p.tile_tab[0], tiles_m);
-  const int n_tiles = tiles_m * p.tiles_n, n_wg = n_tiles * p.parts;
+  const int n_tiles = tiles_m * p.tiles_n;
+  int parts = p.parts;
+  if (GRADE && p.cut.max_parts) parts = p.cut.parts(n_tiles, (float)M * (float)p.N);
+  const int n_wg = n_tiles * parts;
   if ((int)blockIdx.x >= n_wg) return;
   // one contiguous run of workgroups per XCD (they go to the eight XCDs round robin), tiles in it first, then parts:
   // an XCD's tiles share their operand bands in its L2, and with eight parts or more an XCD reads only its part of
@@ -270,8 +294,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
     C = reinterpret_cast<uint8_t*>(C) + (int64_t)e * p.group_stride * (OUT >= 2 ? 4 : 2);
     if ((OUT & 1) && K == 0) return;
   }
-  if (p.parts > 1) {
-    const int slabs = ((K + kTK - 1) / kTK + p.parts - 1) / p.parts;
+  if (parts > 1) {
+    const int slabs = ((K + kTK - 1) / kTK + parts - 1) / parts;
     const int k_begin = part * slabs * kTK;
     A += AT ? (int64_t)k_begin * p.lda : (int64_t)k_begin;
     B += BT ? (int64_t)k_begin * p.ldb : (int64_t)k_begin;
@@ -412,8 +436,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
 
   // a lane holds row m of C and, per accumulator, columns 4 q + {0..3} of a 16-column block
   const int q = lane >> 4, r16 = lane & 15;
-  if (p.parts > 1) {
-    float* const P = p.part_ws + (int64_t)part * p.M * p.N;
+  if (parts > 1) {
+    float* const P = p.part_ws + (int64_t)part * (GRADE && p.cut.max_parts ? tiles_m * TM : p.M) * p.N;
 #pragma unroll
     for (int i = 0; i < kMI; ++i) {
       const int m = m0 + wm + i * 16 + r16;

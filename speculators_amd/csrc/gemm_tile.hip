@@ -67,7 +67,8 @@ static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
   auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE, PICK>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmem, lds_set, fname)) return rc;
   hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE, PICK>),
-                     dim3((unsigned)(p.tiles_m * p.tiles_n * p.parts), (unsigned)groups_y), dim3(64 * WM * WN), kSmem,
+                     dim3((unsigned)std::max(p.tiles_m * p.tiles_n * p.parts, p.cut.max_parts ? p.cut.cap : 0), (unsigned)groups_y),
+                     dim3(64 * WM * WN), kSmem,
                      st, p);
   return check_launch(fname);
 }
@@ -174,12 +175,20 @@ int grouped_tn(const char* fname, const void* a, int64_t lda, const void* b, int
 
 // ------------------------------------------------------------------------------------------ plain products
 // C[m, n .. n + 7] = the sum of the parts of a product whose contraction was cut, in their order, fp32, one rounding.
-// OUT as in gemm_tile_kernel; grade (OUT 0): what the rows of the sum are multiplied by.
+// OUT as in gemm_tile_kernel; grade (OUT 0): what the rows of the sum are multiplied by; cut: the parts were chosen on the
+// device, for tiles of tm x tn (one part: the product has stored its results).
 template <int OUT>
 __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ ws, void* __restrict__ C,
                                                            int64_t ldc, int M_host, int N, int parts,
-                                                           const int32_t* __restrict__ m_live, RowGrade grade) {
+                                                           const int32_t* __restrict__ m_live, RowGrade grade,
+                                                           LiveCut cut, int tm, int tn) {
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
+  if (OUT == 0 && cut.max_parts) {
+    const int tiles_m = (M + tm - 1) / tm;
+    parts = cut.parts(tiles_m * ((N + tn - 1) / tn), (float)M * (float)N);
+    if (parts == 1) return;
+    M_host = tiles_m * tm;
+  }
   const int n8 = N / 8;
   const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (item >= (int64_t)M * n8) return;
@@ -216,10 +225,11 @@ __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restri
 
 template <int OUT>
 static int launch_reduce(const char* fname, const float* ws, void* c, int64_t ldc, int64_t M, int64_t N, int parts,
-                         const int32_t* m_live, hipStream_t st, const RowGrade& grade = RowGrade{}) {
+                         const int32_t* m_live, hipStream_t st, const RowGrade& grade = RowGrade{},
+                         const LiveCut& cut = LiveCut{}, int tm = 1, int tn = 1) {
   const int64_t items = M * (N / 8);
   hipLaunchKernelGGL(parts_reduce_kernel<OUT>, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, ws, c, ldc, (int)M,
-                     (int)N, parts, m_live, grade);
+                     (int)N, parts, m_live, grade, cut, tm, tn);
   return check_launch(fname);
 }
 
@@ -282,8 +292,6 @@ static float predict(const Config& c, int64_t tiles, int slabs) {
   return t;
 }
 
-static float reduce_us(int64_t elements) { return 4.1f + 1.03e-6f * (float)elements; }
-
 // (form 2: b a^T with the count of rows on the device.  No tiles of 192 rows there: the 256 x 256 kernel cuts its contraction
 // by the rows that count, which the host does not know -- 3001 rows x 32000 -> 4096, two thirds of them counting: 516 us
 // in parts, 661 on 192 x 256 tiles.)
@@ -303,7 +311,7 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
       cut = tp > 1 ? rem : 0;
     }
     best.us = predict(c, tiles - cut, slabs);
-    if (cut) best.us += predict(c, cut * tp, (slabs + tp - 1) / tp) + reduce_us(cut * tp * 65536);
+    if (cut) best.us += predict(c, cut * tp, (slabs + tp - 1) / tp) + reduce_us((float)(cut * tp * 65536));
   }
   for (int t = 1; t < (nn ? 7 : form == 2 ? (int)k192x256 : 6); ++t) {
     const Config& c = table[t];
@@ -315,11 +323,19 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
                         tiles * parts > cap))
         break;
       float us = predict(c, tiles * parts, (slabs + parts - 1) / parts);
-      if (parts > 1) us += reduce_us(parts * M * N);
+      if (parts > 1) us += reduce_us((float)(parts * M * N));
       if (us < best.us) best = Choice{t, parts, us};
     }
   }
   return best;
+}
+
+// The most that the parts of a product cut on the device (LiveCut) leave behind, in floats; 0: it is not cut there.
+static int64_t live_cut_floats(const Config& c, int64_t M, int64_t N, int64_t K, int max_parts) {
+  if (max_parts <= 1 || (K + kTK - 1) / kTK < kSplitFrom) return 0;
+  const int64_t tiles_n = (N + c.tn - 1) / c.tn, rows = (M + c.tm - 1) / c.tm * c.tm;
+  if (tiles_n * 2 > kCus * c.per_cu) return 0;
+  return std::min<int64_t>((int64_t)kCus * c.per_cu * c.tm * c.tn, kMaxParts * rows * N);
 }
 
 static Choice choose_tn(int64_t M, int64_t N, int64_t T, bool can_split) {
@@ -333,7 +349,7 @@ static Choice choose_tn(int64_t M, int64_t N, int64_t T, bool can_split) {
     for (int parts = 1; parts <= kTnParts; ++parts) {
       if (parts > 1 && (!can_split || slabs / parts < kMinSlabs || tiles * parts > (int64_t)kCus * c.per_cu)) break;
       float us = predict(c, tiles * parts, (slabs + parts - 1) / parts);
-      if (parts > 1) us += reduce_us(parts * M * N);
+      if (parts > 1) us += reduce_us((float)(parts * M * N));
       if (us < best.us) best = Choice{t, parts, us};
     }
   }
@@ -475,7 +491,8 @@ extern "C" int64_t spx_gemm_auto_workspace_bytes(int form, int64_t M, int64_t N,
   if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1) return 0;
   const tile::Choice c = tile::choose(form, M, N, K, max_parts, can_split(N));
   if (c.tile == tile::kBig) return max_parts > 1 ? spx_gemm_tail_workspace_bytes() : 0;
-  return c.parts > 1 ? (int64_t)c.parts * M * N * (int64_t)sizeof(float) : 0;
+  const int64_t cut = form == 2 && can_split(N) ? tile::live_cut_floats(tile::kNT[c.tile], M, N, K, max_parts) : 0;
+  return std::max(c.parts > 1 ? c.parts * M * N : 0, cut) * (int64_t)sizeof(float);
 }
 
 extern "C" float spx_gemm_auto_us(int form, int64_t M, int64_t N, int64_t K, int32_t max_parts) {
@@ -560,10 +577,18 @@ extern "C" int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void*
   p.part_ws = reinterpret_cast<float*>(workspace);
   p.m_live = m_live;
   p.grade = grade;
+  // The host cuts for all M rows; the parts chosen for the live ones, us: x 32000 -> 2048, 1075 live of 1536 rows 172 -> 141,
+  // 768 of them 162 -> 93, 716 of 1024 98 -> 92, 512 of them 92 -> 69, 620 of 888 98 -> 90; -> 4096, 460 of 1536 345 -> 123; all rows
+  // live: as before.
+  const int64_t floats = tile::live_cut_floats(cfg, M, N, K, max_parts);
+  if (can_split(N) && vec && workspace && floats && workspace_bytes >= floats * (int64_t)sizeof(float)) {
+    const int slabs = (int)((K + tile::kTK - 1) / tile::kTK);
+    p.cut = {std::min(tile::kMaxParts, slabs / tile::kMinSlabs), tile::kCus * cfg.per_cu, slabs, cfg.s0, cfg.s1};
+  }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (int rc = tile::launch_graded(fname, ch.tile, p, st)) return rc;
-  if (ch.parts == 1) return SPX_OK;
-  return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st, grade);
+  if (ch.parts == 1 && !p.cut.max_parts) return SPX_OK;
+  return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st, grade, p.cut, cfg.tm, cfg.tn);
 }
 
 // ------------------------------------------------------------------------------------------ weight gradients
