@@ -767,8 +767,9 @@ int spx_gemm_bf16_nt_rows_split(const void* a, int64_t lda, const void* b, int64
  * spx_vocab_loss_terms_fwd_grad): row m of c is row row[m] of the whole and is multiplied by
  * row_weight[row[m]] * (*scale * factor) in fp32, before its one rounding.  Tiles and parts as spx_gemm_bf16_auto chooses
  * them in form 2 (max_parts: as there; workspace: spx_gemm_auto_workspace_bytes(2, ..) bytes, NULL: no cut), on the
- * 256 x 256 kernel as spx_gemm_bf16_nt_rows_split with split_parts where the workspace holds them (split_parts * M * N
- * floats), else as spx_gemm_bf16_nt_rows.  m_live, row, row_weight and scale are device memory. */
+ * 256 x 256 kernel with the tiles of its last round of live ones in up to split_parts (1 .. 8) parts, as many as the workspace
+ * has room for (a part of a tile: 65536 floats; any size will do).  The smaller tiles choose their parts by the live rows
+ * where the workspace is of that size. m_live, row, row_weight and scale are device memory. */
 int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
                               int64_t N, int64_t K, const int32_t* m_live, const int32_t* row, const float* row_weight,
                               const float* scale, float factor, int32_t max_parts, int32_t split_parts, void* workspace,

@@ -27,6 +27,7 @@
 // (ids are dealt round-robin over the 8 XCDs) works on a compact band of
 // tiles and shares its A / B panels in that XCD's L2.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_tile_api.h"
@@ -110,6 +111,31 @@ __host__ __device__ __forceinline__ void tail_plan(int n_tiles, int cus, int nsl
   if (tp > 1) { first = n_tiles - rem; parts = tp; }
 }
 
+// The same for a product whose rows are counted on the device, and for any last round: as many parts (at most max_parts, each
+// at least 16 slabs, tiles x parts at most `room` partial tiles) as make it shortest.  The times are those of the 256 x 256 tile,
+// as gemm_tile.hip has them, 16 us for a part's start and its 256 KB of partial results, and the pass behind it
+// (reduce_us there); one more part has to promise 3 %.  400 tiles: 256 whole ones, then 144 in 5 parts, 3 / 5 of a round in the
+// place of one.  x 32000, us, all tiles cut in up to 4 parts (where there are at most 512) / so: -> 4096, 6300 live of 9003 rows
+// 1455 / 1300, 4500 of them 1416 / 898, 4200 of 6000 1042 / 867; -> 8192, 2150 of 3072 1020 / 865; -> 2048, 1260 of 1800
+// 173 / 154, 900 of them 152 / 116, 1800 of them 202 / 208; worst 1800 of 3600 200 / 209.
+__device__ __forceinline__ void live_tail_plan(int n_tiles, int cus, int nslab, int max_parts, int room, int& first,
+                                               int& parts) {
+  first = n_tiles;
+  parts = 1;
+  const int rem = n_tiles > 0 ? n_tiles % cus : 0;
+  if (rem == 0) return;
+  auto rounds = [&](int wgs, int slabs) __attribute__((always_inline)) {
+    const int last = wgs % cus;
+    return (float)slabs * ((float)(wgs / cus) * 1.41f + (last ? 1.18f + 0.23f * (float)last / (float)cus : 0.f));
+  };
+  float best = rounds(rem, nslab) + 6.9f;
+  for (int p = 2; p <= max_parts && nslab / p >= 16 && rem * p <= room; ++p) {
+    const float t = rounds(rem * p, (nslab + p - 1) / p) + 16.f * (float)((rem * p + cus - 1) / cus) + 4.1f +
+                    1.03e-6f * 65536.f * (float)(rem * p);
+    if (t < 0.97f * best) { best = t; first = n_tiles - rem; parts = p; }
+  }
+}
+
 // tile index -> (tile row, tile column).  256 consecutive indices (what the chip runs at a time) are a block of
 // 16 x 16 tiles, so that a 256-row band of either operand is used by 16 of the tiles in flight, and the blocks walk
 // along the longer side of the tile grid; 32 consecutive indices (what one XCD runs: see the kernel) are 8 tiles
@@ -162,9 +188,11 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   // K and leave an fp32 partial in part_ws[p]; gemm_splitk_reduce_kernel adds the parts in order
   const int n_tiles = tiles_m * tiles_n;
   // tail_mode: only the tiles of the last, partly filled round are cut (tail_plan); their partials go to
-  // part_ws as whole tiles, [part][tail tile][256][256] fp32, and gemm_tail_reduce_kernel adds them
+  // part_ws as whole tiles, [part][tail tile][256][256] fp32, and gemm_tail_reduce_kernel adds them; kGrade: by
+  // live_tail_plan, with tail_mode partial tiles of room
   int parts = 1, tail_first = n_tiles, tail_parts = 1;
-  if (tail_mode) tail_plan(n_tiles, cus, (K + kTK - 1) / kTK, max_parts, tail_first, tail_parts);
+  if (kGrade && tail_mode) live_tail_plan(n_tiles, cus, (K + kTK - 1) / kTK, max_parts, tail_mode, tail_first, tail_parts);
+  else if (tail_mode) tail_plan(n_tiles, cus, (K + kTK - 1) / kTK, max_parts, tail_first, tail_parts);
   else if (part_ws) parts = choose_k_parts(n_tiles, max_parts, cus, (K + kTK - 1) / kTK);
   const int n_tail = n_tiles - tail_first;
   const int n_wg = tail_mode ? n_tiles + n_tail * (tail_parts - 1) : n_tiles * parts;
@@ -173,10 +201,9 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   {
     constexpr int kRound = 256, kPer = kRound / 8;
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-    // tail_mode with a cut last round: the whole tiles are whole rounds, the parts of the cut tiles are "what
-    // is left" -- dispatched after them (workgroups start in the order of their ids) and everywhere at once
-    const int whole = (tail_mode && tail_parts > 1) ? tail_first : n_wg;
-    const int full = whole / kRound * kRound;
+    // (with a cut last round the whole tiles are whole rounds, and the parts of the cut ones are rounds of their own behind
+    // them: workgroups start in the order of their ids)
+    const int full = n_wg / kRound * kRound;
     if ((int)blockIdx.x < full) {
       pid = (local / kPer) * kRound + xcd * kPer + local % kPer;
     } else {
@@ -567,26 +594,34 @@ __global__ __launch_bounds__(256) void gemm_row_stats_reduce_kernel(const float*
 }
 
 // The tiles of the last round of a product cut by tail_plan: C[tile] = the sum of its parts, in their
-// order, fp32, one rounding.  blockIdx.x = (tail tile, one of kTailSlices bands of 32 rows): 256 threads x 4
-// passes of 8 columns, enough workgroups to fill the chip for the 128 tiles of half a round.
+// order, fp32, one rounding.  A workgroup takes 8 rows (256 threads x 8 columns) of a tile at a time, eight workgroups for every
+// tile that there may be: four times for each where all are there, once where a quarter of them are.
+// kGrade: cut by live_tail_plan for the rows that count, the sums multiplied by their rows' factors.
 constexpr int kTailSlices = 8;
+template <bool kGrade>
 __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const float* __restrict__ part_ws,
                                                                uint16_t* __restrict__ C, int64_t ldc, int M, int N,
                                                                int K, int tiles_m, int tiles_n, int max_parts,
-                                                               int cus) {
+                                                               int cus, int room, const int32_t* __restrict__ m_live,
+                                                               RowGrade grade) {
   int tail_first, tail_parts;
-  tail_plan(tiles_m * tiles_n, cus, (K + kTK - 1) / kTK, max_parts, tail_first, tail_parts);
+  if (kGrade) {
+    M = min(M, max(*m_live, 0));
+    tiles_m = (M + kTM - 1) / kTM;
+    live_tail_plan(tiles_m * tiles_n, cus, (K + kTK - 1) / kTK, max_parts, room, tail_first, tail_parts);
+  } else {
+    tail_plan(tiles_m * tiles_n, cus, (K + kTK - 1) / kTK, max_parts, tail_first, tail_parts);
+  }
   const int n_tail = tiles_m * tiles_n - tail_first;
-  const int tail_idx = (int)blockIdx.x / kTailSlices, slice = (int)blockIdx.x % kTailSlices;
-  if (tail_parts <= 1 || tail_idx >= n_tail) return;
-  int tile_m, tile_n;
-  tile_coords(tail_first + tail_idx, tiles_m, tiles_n, tile_m, tile_n);
-  const int m0 = tile_m * kTM, n0 = tile_n * kTN;
+  if (tail_parts <= 1) return;
   const bool fast = (ldc % 8 == 0) && ((reinterpret_cast<uintptr_t>(C) & 15) == 0);
-  constexpr int kItems = kTM * (kTN / 8) / kTailSlices;
-  for (int it = slice * kItems + threadIdx.x; it < (slice + 1) * kItems; it += 256) {
+  constexpr int kChunks = kTM * (kTN / 8) / 256;
+  for (int c = (int)blockIdx.x; c < n_tail * kChunks; c += (int)gridDim.x) {
+    const int tail_idx = c / kChunks, it = c % kChunks * 256 + (int)threadIdx.x;
+    int tile_m, tile_n;
+    tile_coords(tail_first + tail_idx, tiles_m, tiles_n, tile_m, tile_n);
     const int rr = it / (kTN / 8), cc = (it % (kTN / 8)) * 8;
-    const int m = m0 + rr, n = n0 + cc;
+    const int m = tile_m * kTM + rr, n = tile_n * kTN + cc;
     if (m >= M || n >= N) continue;
     f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
     for (int p = 0; p < tail_parts; ++p) {
@@ -594,6 +629,11 @@ __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const float* __re
       const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
       lo[0] += a[0]; lo[1] += a[1]; lo[2] += a[2]; lo[3] += a[3];
       hi[0] += b[0]; hi[1] += b[1]; hi[2] += b[2]; hi[3] += b[3];
+    }
+    if (kGrade) {
+      const float by = grade.at(m);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) { lo[r] *= by; hi[r] *= by; }
     }
     u32x4 v;
     v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
@@ -614,7 +654,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
                                                                  uint16_t* __restrict__ C, int64_t ldc, int M_host,
                                                                  int N, int K, int tiles_n,
                                                                  const int32_t* __restrict__ m_live, int max_parts,
-                                                                 int cus, RowGrade grade) {
+                                                                 int cus) {
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
   const int parts = choose_k_parts(((M + kTM - 1) / kTM) * tiles_n, max_parts, cus, (K + kTK - 1) / kTK);
   if (parts <= 1) return;
@@ -628,11 +668,6 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
     lo[0] += a[0]; lo[1] += a[1]; lo[2] += a[2]; lo[3] += a[3];
     hi[0] += b[0]; hi[1] += b[1]; hi[2] += b[2]; hi[3] += b[3];
-  }
-  if (grade.row) {
-    const float by = grade.at(m);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) { lo[r] *= by; hi[r] *= by; }
   }
   u32x4 v;
   v.x = pack_bf16x2(lo[0], lo[1]); v.y = pack_bf16x2(lo[2], lo[3]);
@@ -700,7 +735,9 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
   const int cus = compute_units();
   int64_t n_grid = (int64_t)tiles_m * tiles_n * (part_ws ? max_parts : 1);
   int tail_first = tiles_m * tiles_n, tail_parts = 1;
-  if (tail_mode) {
+  if (grade.row) {  // (fewer rows than M may have the larger last round)
+    n_grid = (int64_t)tiles_m * tiles_n + (tail_mode ? std::min<int64_t>(tail_mode, (int64_t)cus * max_parts) : 0);
+  } else if (tail_mode) {
     tail_plan(tiles_m * tiles_n, cus, (int)((K + kTK - 1) / kTK), max_parts, tail_first, tail_parts);
     n_grid = (int64_t)tiles_m * tiles_n + (int64_t)(tiles_m * tiles_n - tail_first) * (tail_parts - 1);
   }
@@ -724,12 +761,19 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
   }
 #undef SPX_GEMM_LAUNCH
   if (int rc = check_launch(fname)) return rc;
+  if (grade.row && !tail_mode) return 0;
+  if (grade.row) {
+    hipLaunchKernelGGL(gemm_tail_reduce_kernel<true>, dim3((unsigned)(std::min(tiles_m * tiles_n, cus - 1) * kTailSlices)),
+                       dim3(256), 0, st, part_ws, reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_m,
+                       tiles_n, max_parts, cus, tail_mode, m_live, grade);
+    return check_launch(fname);
+  }
   if (tail_mode) {
     if (tail_parts > 1) {
-      hipLaunchKernelGGL(gemm_tail_reduce_kernel,
+      hipLaunchKernelGGL(gemm_tail_reduce_kernel<false>,
                          dim3((unsigned)((tiles_m * tiles_n - tail_first) * kTailSlices)), dim3(256), 0, st,
                          part_ws, reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_m, tiles_n,
-                         max_parts, cus);
+                         max_parts, cus, 0, nullptr, grade);
       return check_launch(fname);
     }
     return 0;
@@ -737,7 +781,7 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
   if (part_ws) {
     const int64_t items = M * (N / 8);
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, part_ws,
-                       reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_n, m_live, max_parts, cus, grade);
+                       reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_n, m_live, max_parts, cus);
     return check_launch(fname);
   }
   return 0;
@@ -880,8 +924,9 @@ extern "C" int spx_gemm_bf16_nt_rows(const void* a, int64_t lda, const void* b, 
 
 int spx::nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                         int64_t M, int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws,
-                        int max_parts, void* stream) {
-  return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream, nullptr, nullptr, 0, 0, part_ws,
-                      part_ws ? max_parts : 1, nullptr, 0, 0, grade);
+                        int64_t part_floats, int max_parts, void* stream) {
+  const int room = part_ws && max_parts > 1 ? (int)std::min<int64_t>(part_floats / (kTM * kTN), 1 << 20) : 0;
+  return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream, nullptr, nullptr, 0, 0, room ? part_ws : nullptr,
+                      room ? max_parts : 1, nullptr, 0, room, grade);
 }
 #undef SPX_REQ_FN

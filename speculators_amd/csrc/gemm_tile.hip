@@ -559,9 +559,8 @@ extern "C" int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void*
   const tile::Choice ch = tile::choose(2, M, N, K, max_parts, can_split(N) && vec && workspace);
   const int64_t part = M * N * (int64_t)sizeof(float);
   if (ch.tile == tile::kBig) {
-    const bool cut = split_parts > 1 && can_split(N) && vec && workspace && workspace_bytes >= split_parts * part;
-    return nt_rows_graded(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, grade,
-                          cut ? reinterpret_cast<float*>(workspace) : nullptr, split_parts, stream);
+    return nt_rows_graded(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, grade, reinterpret_cast<float*>(workspace),
+                          workspace ? workspace_bytes / (int64_t)sizeof(float) : 0, split_parts, stream);
   }
   SPX_REQ_FN(ch.parts == 1 || workspace_bytes >= ch.parts * part, "workspace too small");
   const tile::Config& cfg = tile::kNT[ch.tile];

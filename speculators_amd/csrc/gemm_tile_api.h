@@ -16,10 +16,10 @@ struct RowGrade {
   __device__ __forceinline__ float at(int m) const { return weight[row[m]] * (*scale * factor); }
 };
 
-// spx_gemm_bf16_nt_rows (part_ws == nullptr) or spx_gemm_bf16_nt_rows_split with graded rows (gemm_bf16.hip)
+// spx_gemm_bf16_nt_rows with graded rows, its last round cut where part_ws has room (gemm_bf16.hip)
 int nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
-                   int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws, int max_parts,
-                   void* stream);
+                   int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws, int64_t part_floats,
+                   int max_parts, void* stream);
 
 namespace tile {
 

@@ -31,6 +31,8 @@ if not 1 <= SPLIT_PARTS <= 8:
     raise ValueError(f"SPX_GEMM_SPLIT_PARTS must be 1 .. 8, got {SPLIT_PARTS}")
 
 
+# parts the last round's tiles of such a product with graded rows may be cut into, and partial tiles of 256 KB held for them
+LIVE_TAIL_PARTS, LIVE_TAIL_TILES = 8, 1024
 # parts the tiles of a mostly empty last round of a product may be cut into (spx_gemm_bf16_nt_tail); 1 = never
 TAIL_PARTS = int(os.environ.get("SPX_GEMM_TAIL_PARTS", "4"))
 if not 1 <= TAIL_PARTS <= 8:
@@ -159,13 +161,13 @@ def rows_graded(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor, row_of: 
     if b.stride(1) != 1:
         b = b.contiguous()
     big, ws_numel, _ = _plan(2, m, n, k, TAIL_PARTS)
-    if big:  # (as gemm_nt(split=True))
-        few_tiles = -(-m // 256) * -(-n // 256) <= 2 * _CUS
-        ws_numel = SPLIT_PARTS * m * n if SPLIT_PARTS > 1 and few_tiles and n % 8 == 0 and k >= 64 * 16 * 2 else 0
+    parts = LIVE_TAIL_PARTS if SPLIT_PARTS > 1 else 1
+    if big:
+        ws_numel = min(LIVE_TAIL_TILES, parts * -(-m // 256) * -(-n // 256)) * 65536 if parts > 1 and k >= 64 * 16 * 2 else 0
     ws = _split_workspace(a.device, ws_numel) if ws_numel else None
     out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
     _lib.call("spx_gemm_bf16_rows_graded", a, a.stride(0), b, b.stride(0), out, n, m, n, k, m_live, row_of, row_weight, scale,
-              factor, TAIL_PARTS, SPLIT_PARTS, ws, ws.numel() * 4 if ws_numel else 0, _lib.stream_ptr(a.device))
+              factor, TAIL_PARTS, parts, ws, ws.numel() * 4 if ws_numel else 0, _lib.stream_ptr(a.device))
     return out
 
 

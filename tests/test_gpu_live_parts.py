@@ -37,3 +37,31 @@ def test_live_parts_against_float64(m, n, k, live):
         assert rows == 0 or ((c[:rows].double() - want).abs() <= bound).all()
         got.append(c)
     assert torch.equal(*got)
+
+
+# the 256 x 256 kernel: last rounds of 16 tiles behind a whole one, of 160, of one, with room for all, some and no parts
+@pytest.mark.parametrize("n", [4096, 4100])
+@pytest.mark.parametrize("live", [0, 1, 2500, 4097, 4999])
+def test_last_round_of_live_tiles_against_float64(n, live):
+    from speculators_amd import _lib
+
+    m, k = 5000, 4104
+    assert _lib.load().spx_gemm_auto_tile(2, m, n, k, 4) == 0
+    g = torch.Generator(device="cuda").manual_seed(live)
+    a = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    b = torch.randn(n, k, device="cuda", generator=g).bfloat16()
+    weight = torch.rand(m, device="cuda", generator=g) + 0.5
+    want = (a[:live].double() @ b.double().t()) * weight[:live].double().unsqueeze(1)
+    bound = 2 ** -8 * torch.exp2(want.abs().clamp_min(1e-30).log2().floor())
+    bound = bound + 2 ** -22 * (a[:live].double().abs() @ b.double().abs().t()) * weight[:live].double().unsqueeze(1)
+    order = torch.arange(m, device="cuda", dtype=torch.int32)
+    count = torch.tensor([live], dtype=torch.int32, device="cuda")
+    for room in (1024, 100, 0):
+        ws = torch.full((room * 65536 + 1024,), 3.0, device="cuda")
+        for _ in range(2):
+            c = torch.full((m, n + 8), 2.0, dtype=torch.bfloat16, device="cuda")
+            _lib.call("spx_gemm_bf16_rows_graded", a, k, b, k, c, n + 8, m, n, k, count, order, weight,
+                      torch.ones((), device="cuda"), 1.0, 4, 8, ws if room else None, room * 65536 * 4,
+                      _lib.stream_ptr(a.device))
+            assert (ws[room * 65536:] == 3).all() and (c[live:] == 2).all() and (c[:, n:] == 2).all()
+            assert live == 0 or ((c[:live, :n].double() - want).abs() <= bound).all()
