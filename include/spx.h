@@ -319,23 +319,27 @@ int spx_mask_row_lists(const void* mask, int mask_kind, int64_t rows, int32_t* r
  * arg-max of every draft row, hits = it is the target's.  grad_logits (or NULL, with the four lists then): the row of
  * step k at the live target of rank i is row i * steps + k, softmax(x) - softmax(y) (kl) or - onehot(argmax y) (ce);
  * zeros where k exceeds the target's row.  row_slot [steps][T] = that row or -1, slot_row its inverse, *slots = live * steps,
- * row_weight = mask * inv[k].  With grad_logits the losses of masked rows behind step 0 are written as 0.
+ * row_weight = mask * inv[k].  With grad_logits the losses of masked rows are written as 0 (masked_first: behind step 0).
+ * terms (0: the one loss `op`): a set of kl, ce and tv (bit op) with their weights in term_weights[op] (host memory, 5 elements), as
+ * spx_vocab_loss_terms_fwd_grad takes them: loss [terms][steps][T], unweighted, the gradient that of their weighted sum.
  *
- * spx_loss_steps_total: out[k][8] as spx_ttt_step_total leaves it for every step, prev_correct (or NULL) [T] advanced over
- * all steps, total = the sum of out[k][6].  partials: spx_loss_steps_partials floats. */
+ * spx_loss_steps_total: out[k][8] as spx_ttt_step_total leaves it for every step (terms: out[k][18] as spx_ttt_step_terms),
+ * prev_correct (or NULL) [T] advanced over all steps, total = the sum of out[k][6].  partials: spx_loss_steps_partials floats. */
 #define SPX_LOSS_STEPS_MAX 32
 int spx_loss_steps_mask(const void* mask, int mask_kind, int64_t T, int32_t steps, const float* step_weights,
                         int32_t* row_map, int32_t* live, float* inv, float* mask_sum, int32_t* full, int32_t* ticket,
                         void* stream);
-int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld_logits, const void* targets, int64_t ld_targets,
-                        const int32_t* argmax_target, int64_t T, int64_t vocab, int32_t steps, int32_t first, int32_t end,
-                        const void* mask, int mask_kind, const float* inv, const int32_t* row_map, const int32_t* live,
-                        float* loss, int64_t* tokens, uint8_t* hits, int32_t* row_slot, int32_t* slot_row, int32_t* slots,
-                        float* row_weight, void* grad_logits, int64_t ld_grad, void* stream);
-int64_t spx_loss_steps_partials(int64_t T, int32_t steps);
+int spx_loss_steps_pass(int op, int32_t terms, const float* term_weights, const void* const* logits, int64_t ld_logits,
+                        const void* targets, int64_t ld_targets, const int32_t* argmax_target, int64_t T, int64_t vocab,
+                        int32_t steps, int32_t first, int32_t end, int32_t masked_first, const void* mask, int mask_kind,
+                        const float* inv, const int32_t* row_map, const int32_t* live, float* loss, int64_t* tokens,
+                        uint8_t* hits, int32_t* row_slot, int32_t* slot_row, int32_t* slots, float* row_weight,
+                        void* grad_logits, int64_t ld_grad, void* stream);
+int64_t spx_loss_steps_partials(int64_t T, int32_t steps, int32_t terms);
 int spx_loss_steps_total(const float* loss, const uint8_t* hits, const void* mask, int mask_kind, void* prev_correct,
-                         int prev_kind, int64_t T, int32_t steps, float factor, const float* inv, const float* mask_sum,
-                         const int32_t* full, float* partials, int32_t* ticket, float* out, float* total, void* stream);
+                         int prev_kind, int64_t T, int32_t steps, float factor, int32_t terms, const float* term_weights,
+                         const float* inv, const float* mask_sum, const int32_t* full, float* partials, int32_t* ticket,
+                         float* out, float* total, void* stream);
 
 /* Draft tokens: out[i] = known[i] for i < n (int32 arg-maxes of a loss pass, widened), out[n + j] = the first
  * index of the maximum of row j < tail of rows[tail, vocab] (bf16 / f32, row stride ld). */

@@ -49,10 +49,10 @@ SIGNATURES["spx_ttt_step_terms"] = [_I32, _P, _P, _P, _I, _I64, _F, _P, _P, _P, 
 SIGNATURES["spx_mask_row_map"] = [_P, _I, _I64, _P, _P, _P, _P]
 SIGNATURES["spx_mask_row_lists"] = [_P, _I, _I64, _P, _P, _P, _P, _P]
 SIGNATURES["spx_loss_steps_mask"] = [_P, _I, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _P]
-SIGNATURES["spx_loss_steps_pass"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I32, _I32, _I32, _P, _I, _P, _P, _P, _P, _P, _P,
-                                     _P, _P, _P, _P, _P, _I64, _P]
-SIGNATURES["spx_loss_steps_partials"] = [_I64, _I32]
-SIGNATURES["spx_loss_steps_total"] = [_P, _P, _P, _I, _P, _I, _I64, _I32, _F, _P, _P, _P, _P, _P, _P, _P, _P]
+SIGNATURES["spx_loss_steps_pass"] = [_I, _I32, _P, _P, _I64, _P, _I64, _P, _I64, _I64, _I32, _I32, _I32, _I32, _P, _I, _P, _P,
+                                     _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _P]
+SIGNATURES["spx_loss_steps_partials"] = [_I64, _I32, _I32]
+SIGNATURES["spx_loss_steps_total"] = [_P, _P, _P, _I, _P, _I, _I64, _I32, _F, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P]
 SIGNATURES["spx_row_tokens"] = [_P, _I64, _P, _I64, _I64, _I64, _I, _P, _P]
 SIGNATURES["spx_span_attn_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _I32, _I32, _I32, _F, _P, _P,
                                    _P, _I64, _P]
@@ -149,7 +149,7 @@ SIGNATURES["spx_gemm_auto_us"] = [_I, _I64, _I64, _I64, _I32]
 SIGNATURES["spx_gemm_auto_tile"] = [_I, _I64, _I64, _I64, _I32]
 SIGNATURES["spx_gemm_bf16_auto"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P]
 SIGNATURES["spx_stage_upload"] = [_P, _I64, _P, _P, _I64, _I32, _P]
-RESTYPES = {"spx_gemm_auto_workspace_bytes": c_int64, "spx_gemm_tn_workspace_bytes": c_int64, "spx_gemm_auto_us": c_float, "spx_moe_sort_workspace_bytes": c_int64, "spx_gemm_grouped_workspace_bytes": c_int64, "spx_gemm_tail_workspace_bytes": c_int64, "spx_gemm_stats_workspace_bytes": c_int64, "spx_gemm_split_workspace_bytes": c_int64, "spx_ttt_attn_workspace_bytes": c_int64, "spx_ttt_attn_fwd_static_max_bytes": c_int64, "spx_dflash_attn_workspace_bytes": c_int64,
+RESTYPES = {"spx_gemm_auto_workspace_bytes": c_int64, "spx_gemm_tn_workspace_bytes": c_int64, "spx_gemm_auto_us": c_float, "spx_moe_sort_workspace_bytes": c_int64, "spx_loss_steps_partials": c_int64, "spx_gemm_grouped_workspace_bytes": c_int64, "spx_gemm_tail_workspace_bytes": c_int64, "spx_gemm_stats_workspace_bytes": c_int64, "spx_gemm_split_workspace_bytes": c_int64, "spx_ttt_attn_workspace_bytes": c_int64, "spx_ttt_attn_fwd_static_max_bytes": c_int64, "spx_dflash_attn_workspace_bytes": c_int64,
             "spx_rmsnorm_bwd_slots": c_int64}
 
 _lib = None

@@ -1284,10 +1284,14 @@ __device__ __forceinline__ T wave_all(T v, Op op) {
 // row runs beside the traffic of its neighbour.  Where r < k there is no such draft row, and the workgroup takes row T - k + r
 // instead, one of the k last, which have no target: its arg-max is a draft token like any other.  So every
 // (step, row) is met once.
-//   loss, tokens, hits, row_of_map, row_weight: [steps][T], indexed by draft row; grad and row_slot by slot, K a live
-//   target: slot = rank of the target among the live ones * K + k (k > r: a row of zeros, of weight zero).
+//   loss, tokens, hits, row_slot, row_weight: [steps][T] (a loss of several terms: [term][steps][T]), indexed by draft row;
+//   grad and slot_row by slot, K a live target: slot = rank of the target among the live ones * K + k (k > r: a row of zeros,
+//   of weight zero).
+// TERMS: a weighted sum of kl, ce and tv, as loss_terms_grad_kernel takes it (OP: KL if that is one of them, else CE): a second
+// walk over the registers where tv is a term, and the gradient of the sum.  (rkl and jsd need registers that are not there.)
 // kl, 7 steps of 4096 rows of 32000, 70 % live: a pass a step 1002 us, so 719 (4.7 TB/s; 5.3 for ce: the exponentials of kl
-// take as long as its traffic).  5 steps of 1999 rows without gradient 320 -> 208.
+// take as long as its traffic).  5 steps of 1999 rows without gradient 320 -> 208; {"ce": 0.1, "tv": 0.9}, 3 steps of 3001 407 ->
+// 338.
 struct StepsArgs {
   const uint16_t* logits[SPX_LOSS_STEPS_MAX];  // [T, vocab] each
   int64_t ld;
@@ -1295,6 +1299,8 @@ struct StepsArgs {
   int64_t ld_targets;
   const int32_t* argmax_target;
   int T, vocab, steps, k0, k1;  // this launch: steps k0 .. k1 - 1 of `steps`
+  int masked_first;             // GRAD: the first step's masked rows are formed, too
+  LossTerms tm;                 // TERMS
   const void* mask;
   int mask_kind;
   const float* inv;             // [steps]: weight of a step's masked mean over the sum of its mask
@@ -1311,8 +1317,9 @@ struct StepsArgs {
   int64_t ld_grad;
 };
 
-template <int OP, bool GRAD>
+template <int OP, bool GRAD, bool TERMS = false>
 __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void loss_steps_kernel(StepsArgs a) {
+  constexpr bool kY = OP == SPX_LOSS_KL || TERMS;  // the target row is needed at every step
   const int r = blockIdx.x, tid = threadIdx.x, T = a.T;
   const int nchunks = a.vocab >> 3;
   const int rank = GRAD ? a.row_map[r] : -1;
@@ -1339,6 +1346,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
   }
   struct Part { float m, z, a, b; int i; };
   __shared__ Part part[2][kFgWaves];
+  __shared__ float second[2][kFgWaves];
   int turn = 0;
   // every thread's (maximum, first index of it, sum of 2^(x' - max x'), sum) -> the workgroup's
   auto reduce = [&](float& best, int& at, float& z, float& sum, bool soft) __attribute__((always_inline)) {
@@ -1402,9 +1410,9 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
       float y[8];
       unpack(yr[j], y);
       const float cy = largest(y, c << 3, best, label);
-      if (OP != SPX_LOSS_CE) soften(y, cy, m, z);
+      if (kY) soften(y, cy, m, z);
     }
-    reduce(best, label, z, none, OP != SPX_LOSS_CE);
+    reduce(best, label, z, none, kY);
     lt2 = z;
   } else {
     label = a.argmax_target[r];
@@ -1420,16 +1428,18 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     asm volatile("" : "+v"(label));
 #pragma unroll
     for (int j = 0; j < kFgChunks; ++j)
-      if (OP == SPX_LOSS_KL) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+      if (kY) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
     // (a masked row's loss enters no mean: behind the first step it is not formed where gradients are)
-    const bool soft = !tail && (!GRAD || live || k == 0);
+    const bool soft = !tail && (!GRAD || live || (k == 0 && a.masked_first));
     const bool more = k + 1 < a.k1;
     const uint16_t* const nrow = more ? a.logits[k + 1] + (int64_t)row_of(k + 1) * a.ld : nullptr;
-    const bool early = more && !(GRAD && live);  // the row is read once: its registers are free chunk by chunk
+    const int tm = TERMS ? a.tm.mask : 0;
+    const bool has_tv = tm >> SPX_LOSS_TV & 1, walk2 = TERMS && soft && has_tv;
+    const bool early = more && !(GRAD && live) && !walk2;  // the row is read once: its registers are free chunk by chunk
     float best = -INFINITY, m = kNegBig, z = 0.f, sum = 0.f;
     int at = 0x7fffffff;
     float xt = 0.f;
-    if (OP == SPX_LOSS_CE && tid == 0) xt = load1(xrow + label);
+    if ((OP == SPX_LOSS_CE || TERMS) && tid == 0) xt = load1(xrow + label);
 #pragma unroll
     for (int j = 0; j < kFgChunks; ++j) {
       const int c = tid + j * kFgThreads;
@@ -1449,11 +1459,53 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
       }
     }
     reduce(best, at, z, sum, soft);
+    float sum_v = 0.f, ext_v = 0.f;
+    if (walk2) {
+#pragma unroll
+      for (int j = 0; j < kFgChunks; ++j) {
+        asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
+        asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+      }
+#pragma unroll
+      for (int j = 0; j < kFgChunks; ++j) {
+        const int c = tid + j * kFgThreads;
+        if (c >= nchunks) continue;
+        float x[8], y[8];
+        unpack(xr[j], x);
+        unpack(yr[j], y);
+        if (more && !(GRAD && live)) xr[j] = ld16(nrow + ((int64_t)c << 3));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float dp = fast_exp2(fmaf(x[i], kLog2e, -z)), tp = fast_exp2(fmaf(y[i], kLog2e, -lt2));
+          sum_v += fminf(dp, tp);
+          ext_v += dp <= tp ? dp : 0.f;
+        }
+      }
+      const auto add = [](float x, float y) { return x + y; };
+      sum_v = wave_all(sum_v, add);
+      ext_v = wave_all(ext_v, add);
+      if ((tid & 63) == 0) { second[0][tid >> 6] = sum_v; second[1][tid >> 6] = ext_v; }
+      __syncthreads();  // (the next writes come behind the next step's reduction, its barrier behind these reads)
+      sum_v = ext_v = 0.f;
+#pragma unroll
+      for (int w = 0; w < kFgWaves; ++w) { sum_v += second[0][w]; ext_v += second[1][w]; }
+    }
     if (tid == 0) {
       const int64_t g = (int64_t)k * T + t;
-      float row_loss = 0.f;
-      if (soft) row_loss = OP == SPX_LOSS_KL ? sum - lt2 * kLn2 + z * kLn2 : z * kLn2 - xt;
-      a.loss[g] = row_loss;
+      const float kl = sum - lt2 * kLn2 + z * kLn2, ce = z * kLn2 - xt;
+      if (TERMS) {
+        int64_t at_term = g;
+        auto put = [&](int op, float v) {
+          if (!(tm >> op & 1)) return;
+          a.loss[at_term] = soft ? v : 0.f;
+          at_term += (int64_t)a.steps * T;
+        };
+        put(SPX_LOSS_KL, kl);
+        put(SPX_LOSS_CE, ce);
+        put(SPX_LOSS_TV, 1.f - sum_v);
+      } else {
+        a.loss[g] = soft ? (OP == SPX_LOSS_KL ? kl : ce) : 0.f;
+      }
       a.tokens[g] = at;
       a.hits[g] = at == label;
       if (GRAD) {
@@ -1469,8 +1521,12 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {  // (the packed chunks are what stays in registers between the passes)
         asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
-        if (OP == SPX_LOSS_KL) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+        if (kY) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
       }
+      // TERMS: every term's gradient is the draft probability times a factor, less w_kl times the target's and w_ce at the label
+      const float w_ce = TERMS ? a.tm.w[SPX_LOSS_CE] : 0.f, w_kl = TERMS ? a.tm.w[SPX_LOSS_KL] : 0.f;
+      const float w_tv = TERMS && has_tv ? a.tm.w[SPX_LOSS_TV] : 0.f;
+      const float base_f = w_ce + (OP == SPX_LOSS_KL ? w_kl : 0.f), above = fmaf(w_tv, ext_v, base_f), below = above - w_tv;
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {
         const int c = tid + j * kFgThreads;
@@ -1478,13 +1534,27 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
         const int base = c << 3;
         float x[8], y[8], o[8];
         unpack(xr[j], x);
-        if (OP == SPX_LOSS_KL) unpack(yr[j], y);
+        if (kY) unpack(yr[j], y);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float dp = fast_exp2(fmaf(x[i], kLog2e, cd));
-          if (OP == SPX_LOSS_CE) o[i] = dp - ((base + i) == label ? 1.f : 0.f);
-          else o[i] = dp - fast_exp2(fmaf(y[i], kLog2e, ct));
-          if (tail) o[i] = 0.f;
+          if (TERMS) {
+            const float tp = fast_exp2(fmaf(y[i], kLog2e, ct));
+            o[i] = dp * (dp <= tp ? below : above);
+            if (OP == SPX_LOSS_KL) o[i] = fmaf(-w_kl, tp, o[i]);
+          } else if (OP == SPX_LOSS_CE) {
+            o[i] = dp - ((base + i) == label ? 1.f : 0.f);
+          } else {
+            o[i] = dp - fast_exp2(fmaf(y[i], kLog2e, ct));
+          }
+        }
+        if (TERMS && c == label >> 3) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) o[i] -= i == (label & 7) ? w_ce : 0.f;
+        }
+        if (tail) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) o[i] = 0.f;
         }
         store8_vec<uint16_t>(grow + base, o);
         if (more) xr[j] = ld16(nrow + base);
@@ -1530,45 +1600,56 @@ __global__ __launch_bounds__(1024) void steps_mask_kernel(const void* __restrict
 }
 
 // Behind the row passes: the acceptance chain along a draft row's steps, every step's masked mean and counts (as
-// ttt_step_reduce_kernel leaves them in out[k][8]) and the loss.  A thread owns a draft row; the workgroups' partial sums are
+// ttt_step_reduce_kernel leaves them in out[k][8], for several terms ttt_step_terms_kernel in out[k][18]) and the loss.  A thread owns a draft row; the workgroups' partial sums are
 // added in their order by the one that arrives last, which resets nothing and waits for nothing.
 constexpr int kStepsRows = 256;
 __global__ __launch_bounds__(kStepsRows) void steps_total_kernel(
     const float* __restrict__ loss, const uint8_t* __restrict__ hits, const void* __restrict__ mask, int mask_kind,
-    void* prev, int prev_kind, int T, int steps, float factor, const float* __restrict__ inv, const float* __restrict__ msum,
+    void* prev, int prev_kind, int T, int steps, float factor, LossTerms tm, const float* __restrict__ inv, const float* __restrict__ msum,
     const int32_t* __restrict__ full, float* __restrict__ partial, int32_t* __restrict__ ticket, float* __restrict__ out,
     float* __restrict__ total) {
-  __shared__ float ls[kStepsRows / 64][SPX_LOSS_STEPS_MAX];
+  __shared__ float ls[kStepsRows / 64][SPX_LOSS_STEPS_MAX][5];
   __shared__ int cs[kStepsRows / 64][SPX_LOSS_STEPS_MAX][2];
   __shared__ int last;
   __shared__ float parts[SPX_LOSS_STEPS_MAX];
   const int t = blockIdx.x * kStepsRows + threadIdx.x, wave = threadIdx.x >> 6;
+  const int n = tm.mask ? __popc(tm.mask) : 1, values = n + 2;
   bool was = t < T && (!prev || mask_value(prev, prev_kind, t) != 0.f);
   for (int k = 0; k < steps; ++k) {
-    float l = 0.f;
+    float l[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     bool good = false, chained = false;
     if (t < T - k) {
       const float m = mask_value(mask, mask_kind, t + k);
-      l = fmaf(loss[(int64_t)k * T + t], m, 0.f);
+#pragma unroll
+      for (int u = 0; u < 5; ++u)
+        if (u < n) l[u] = loss[((int64_t)u * steps + k) * T + t] * m;
       chained = was;
       was = was && hits[(int64_t)k * T + t];
       good = was && m != 0.f;
     }
-    l = wave_sum(l);
+#pragma unroll
+    for (int u = 0; u < 5; ++u)
+      if (u < n) {
+        l[u] = wave_sum(l[u]);
+        if ((threadIdx.x & 63) == 0) ls[wave][k][u] = l[u];
+      }
     const int correct = __popcll(__ballot(good)), cond = __popcll(__ballot(chained));
-    if ((threadIdx.x & 63) == 0) { ls[wave][k] = l; cs[wave][k][0] = correct; cs[wave][k][1] = cond; }
+    if ((threadIdx.x & 63) == 0) { cs[wave][k][0] = correct; cs[wave][k][1] = cond; }
   }
   if (prev && t < T) store_flag(prev, prev_kind, t, was);
   __syncthreads();
   if ((int)threadIdx.x < steps) {
     const int k = threadIdx.x;
-    float l = 0.f;
     int c = 0, d = 0;
-    for (int w = 0; w < kStepsRows / 64; ++w) { l += ls[w][k]; c += cs[w][k][0]; d += cs[w][k][1]; }
-    float* const p = partial + ((int64_t)blockIdx.x * steps + k) * 3;
-    __hip_atomic_store(p, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(p + 1, __int_as_float(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(p + 2, __int_as_float(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int w = 0; w < kStepsRows / 64; ++w) { c += cs[w][k][0]; d += cs[w][k][1]; }
+    float* const p = partial + ((int64_t)blockIdx.x * steps + k) * values;
+    __hip_atomic_store(p, __int_as_float(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, __int_as_float(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int u = 0; u < n; ++u) {
+      float l = 0.f;
+      for (int w = 0; w < kStepsRows / 64; ++w) l += ls[w][k][u];
+      __hip_atomic_store(p + 2 + u, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   __threadfence();
   __syncthreads();
@@ -1578,21 +1659,40 @@ __global__ __launch_bounds__(kStepsRows) void steps_total_kernel(
   if (!last) return;
   if ((int)threadIdx.x < steps) {
     const int k = threadIdx.x;
-    float l = 0.f;
+    float l[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     int c = 0, d = 0;
     for (int b = 0; b < (int)gridDim.x; ++b) {
-      const float* const p = partial + ((int64_t)b * steps + k) * 3;
-      l += __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      c += __float_as_int(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      d += __float_as_int(__hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      const float* const p = partial + ((int64_t)b * steps + k) * values;
+      c += __float_as_int(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      d += __float_as_int(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+      for (int u = 0; u < 5; ++u)
+        if (u < n) l[u] += __hip_atomic_load(p + 2 + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    float* const o = out + 8 * k;
-    o[0] = l * inv[k];
+    float* const o = out + (tm.mask ? 18 : 8) * k;
+    float sum = l[0] * inv[k];
+    if (tm.mask) {
+      sum = 0.f;
+      int u = 0;
+#pragma unroll
+      for (int op = 0; op < 5; ++op) {
+        float mean = 0.f;
+        if (tm.mask >> op & 1) {
+#pragma unroll
+          for (int v = 0; v < 5; ++v) mean = v == u ? l[v] * inv[k] : mean;
+          sum = fmaf(tm.w[op], mean, sum);
+          ++u;
+        }
+        o[8 + op] = mean;
+        o[13 + op] = 1.f;
+      }
+    }
+    o[0] = sum;
     o[1] = o[3] = (float)c;
     o[2] = (float)full[k];
     o[4] = (float)d;
     o[5] = msum[k];
-    o[6] = parts[k] = l * inv[k] * factor;
+    o[6] = parts[k] = sum * factor;
     o[7] = 1.f;
   }
   __syncthreads();
@@ -2153,17 +2253,19 @@ extern "C" int spx_loss_steps_mask(const void* mask, int mask_kind, int64_t T, i
   return check_launch(__func__);
 }
 
-extern "C" int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld_logits, const void* targets,
+extern "C" int spx_loss_steps_pass(int op, int32_t terms, const float* term_weights, const void* const* logits, int64_t ld_logits, const void* targets,
                                    int64_t ld_targets, const int32_t* argmax_target, int64_t T, int64_t vocab,
-                                   int32_t steps, int32_t first, int32_t end, const void* mask, int mask_kind,
-                                   const float* inv, const int32_t* row_map, const int32_t* live, float* loss,
+                                   int32_t steps, int32_t first, int32_t end, int32_t masked_first, const void* mask,
+                                   int mask_kind, const float* inv, const int32_t* row_map, const int32_t* live, float* loss,
                                    int64_t* tokens, uint8_t* hits, int32_t* row_slot, int32_t* slot_row, int32_t* slots,
                                    float* row_weight, void* grad_logits, int64_t ld_grad, void* stream) {
-  SPX_REQUIRE(op == SPX_LOSS_KL || op == SPX_LOSS_CE, "built for kl and ce");
+  constexpr int kTerms = 1 << SPX_LOSS_KL | 1 << SPX_LOSS_CE | 1 << SPX_LOSS_TV;
+  SPX_REQUIRE(terms ? terms_ok(terms, term_weights) && !(terms & ~kTerms) : op == SPX_LOSS_KL || op == SPX_LOSS_CE,
+              "kl, ce or a set of kl, ce and tv with their weights");
   SPX_REQUIRE(steps_ok(T, steps) && first >= 0 && first < end && end <= steps, "1 .. 32 steps, no more than rows");
   SPX_REQUIRE(vocab > 0 && vocab % 8 == 0 && vocab <= (int64_t)kFgThreads * kFgChunks * 8,
               "vocab must be a multiple of 8, at most 32768");
-  SPX_REQUIRE(targets || (op == SPX_LOSS_CE && argmax_target), "no targets");
+  SPX_REQUIRE(targets || (!terms && op == SPX_LOSS_CE && argmax_target), "no targets");
   SPX_REQUIRE(ld_logits >= vocab && ld_logits % 8 == 0 && (!targets || (ld_targets >= vocab && ld_targets % 8 == 0)) &&
                   (!grad_logits || (ld_grad >= vocab && ld_grad % 8 == 0)),
               "row strides must be multiples of 8 elements, at least vocab");
@@ -2181,6 +2283,8 @@ extern "C" int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld
   a.ld_targets = ld_targets;
   a.argmax_target = argmax_target;
   a.T = (int)T; a.vocab = (int)vocab; a.steps = steps; a.k0 = first; a.k1 = end;
+  a.masked_first = masked_first;
+  a.tm = terms ? loss_terms(terms, term_weights) : LossTerms{};
   a.mask = mask; a.mask_kind = mask_kind; a.inv = inv;
   a.row_map = row_map; a.live = live;
   a.loss = loss; a.tokens = tokens; a.hits = hits;
@@ -2189,27 +2293,31 @@ extern "C" int spx_loss_steps_pass(int op, const void* const* logits, int64_t ld
   a.ld_grad = ld_grad;
   const dim3 grid((unsigned)T), block(kFgThreads);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-#define SPX_SP(OPV, G) hipLaunchKernelGGL((loss_steps_kernel<OPV, G>), grid, block, 0, st, a)
-  if (op == SPX_LOSS_KL) { if (grad_logits) SPX_SP(SPX_LOSS_KL, true); else SPX_SP(SPX_LOSS_KL, false); }
+#define SPX_SP(...) hipLaunchKernelGGL((loss_steps_kernel<__VA_ARGS__>), grid, block, 0, st, a)
+  if (terms >> SPX_LOSS_KL & 1) { if (grad_logits) SPX_SP(SPX_LOSS_KL, true, true); else SPX_SP(SPX_LOSS_KL, false, true); }
+  else if (terms) { if (grad_logits) SPX_SP(SPX_LOSS_CE, true, true); else SPX_SP(SPX_LOSS_CE, false, true); }
+  else if (op == SPX_LOSS_KL) { if (grad_logits) SPX_SP(SPX_LOSS_KL, true); else SPX_SP(SPX_LOSS_KL, false); }
   else { if (grad_logits) SPX_SP(SPX_LOSS_CE, true); else SPX_SP(SPX_LOSS_CE, false); }
 #undef SPX_SP
   return check_launch(__func__);
 }
 
-extern "C" int64_t spx_loss_steps_partials(int64_t T, int32_t steps) {
-  return T <= 0 || steps <= 0 ? 0 : (T + kStepsRows - 1) / kStepsRows * steps * 3;
+extern "C" int64_t spx_loss_steps_partials(int64_t T, int32_t steps, int32_t terms) {
+  return T <= 0 || steps <= 0 ? 0 : (T + kStepsRows - 1) / kStepsRows * steps * (2 + (terms > 0 ? __builtin_popcount(terms) : 1));
 }
 
 extern "C" int spx_loss_steps_total(const float* loss, const uint8_t* hits, const void* mask, int mask_kind,
                                     void* prev_correct, int prev_kind, int64_t T, int32_t steps, float factor,
-                                    const float* inv, const float* mask_sum, const int32_t* full, float* partials,
+                                    int32_t terms, const float* term_weights, const float* inv, const float* mask_sum, const int32_t* full, float* partials,
                                     int32_t* ticket, float* out, float* total, void* stream) {
   SPX_REQUIRE(steps_ok(T, steps), "1 .. 32 steps, no more than rows");
+  SPX_REQUIRE(!terms || terms_ok(terms, term_weights), "terms must be a set of loss ops with their weights");
   SPX_REQUIRE(loss && hits && mask && inv && mask_sum && full && partials && ticket && out && total, "null buffer");
   SPX_REQUIRE(kind_ok(mask_kind) && (!prev_correct || kind_ok(prev_kind)), "unknown element kind");
   hipLaunchKernelGGL(steps_total_kernel, dim3((unsigned)((T + kStepsRows - 1) / kStepsRows)), dim3(kStepsRows), 0,
                      reinterpret_cast<hipStream_t>(stream), loss, hits, mask, mask_kind, prev_correct, prev_kind, (int)T,
-                     steps, factor, inv, mask_sum, full, partials, ticket, out, total);
+                     steps, factor, terms ? loss_terms(terms, term_weights) : LossTerms{}, inv, mask_sum, full, partials, ticket,
+                     out, total);
   return check_launch(__func__);
 }
 

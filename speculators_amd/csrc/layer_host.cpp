@@ -453,37 +453,52 @@ PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // The loss of all steps of a TTT loop (spx_loss_steps_*).  What its launches share lies in two buffers:
 struct LossSteps {
   int64_t T, steps;
+  int32_t terms = 0;  // a set of ops with their weights (0: one loss)
+  float weights[5];
   int32_t *row_map, *live, *slots, *ticket, *full, *row_slot, *slot_row;
   float *inv, *mask_sum, *loss, *row_weight, *partials;
   static int64_t ints(int64_t T, int64_t steps) { return T + 3 + steps + 2 * steps * T; }
-  static int64_t floats_of(int64_t T, int64_t steps) { return 2 * steps + 2 * steps * T + spx_loss_steps_partials(T, (int32_t)steps); }
-  LossSteps(const Tensor& i, const Tensor& f, int64_t T_, int64_t steps_) : T(T_), steps(steps_) {
+  int64_t losses() const { return (terms ? __builtin_popcount(terms) : 1) * steps * T; }
+  int64_t all_floats() const { return 2 * steps + steps * T + losses() + spx_loss_steps_partials(T, (int32_t)steps, terms); }
+  LossSteps(int64_t T_, int64_t steps_, PyObject* term_weights) : T(T_), steps(steps_) {  // None or five numbers, 0: no such term
+    if (term_weights == Py_None) return;
+    TORCH_CHECK_TYPE(PyTuple_Check(term_weights) && PyTuple_GET_SIZE(term_weights) == 5, "five term weights or None");
+    for (int op = 0; op < 5; ++op) {
+      PyObject* const w = PyTuple_GET_ITEM(term_weights, op);
+      weights[op] = 0.f;
+      if (w == Py_None) continue;
+      terms |= 1 << op;
+      weights[op] = (float)PyFloat_AsDouble(w);
+      if (PyErr_Occurred()) throw python_error();
+    }
+  }
+  void bind(const Tensor& i, const Tensor& f) {
     TORCH_CHECK_VALUE(i.scalar_type() == at::kInt && f.scalar_type() == at::kFloat && i.is_contiguous() && f.is_contiguous() &&
-                          i.numel() == ints(T, steps) && f.numel() == floats_of(T, steps),
+                          i.numel() == ints(T, steps) && f.numel() == all_floats(),
                       "the buffers of loss_steps_begin for ", T, " rows and ", steps, " steps");
     row_map = i.mutable_data_ptr<int32_t>();
     live = row_map + T; slots = live + 1; ticket = slots + 1; full = ticket + 1; row_slot = full + steps;
     slot_row = row_slot + steps * T;
     inv = f.mutable_data_ptr<float>();
-    mask_sum = inv + steps; loss = mask_sum + steps; row_weight = loss + steps * T; partials = row_weight + steps * T;
+    mask_sum = inv + steps; row_weight = mask_sum + steps; loss = row_weight + steps * T; partials = loss + losses();
   }
 };
 
-// (mask, its kind, the steps' weights ..) -> (integers, floats; views: live slots, row -> slot, slot -> row, row weights)
+// (mask, its kind, term weights or None, the steps' weights ..) -> (integers, floats; views: live slots, row -> slot, slot -> row, row weights)
 PyObject* spx_layer_loss_steps_begin(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  const int64_t steps = n - 2;
+  const int64_t steps = n - 3;
   TORCH_CHECK_TYPE(steps >= 1 && steps <= SPX_LOSS_STEPS_MAX, "loss_steps_begin takes 1 .. 32 step weights");
   Args x("loss_steps_begin", args, n, n);
   const Tensor& mask = x.tensor();
-  const int64_t kind = x.integer();
+  const int64_t kind = x.integer(), T = mask.numel();
+  LossSteps s(T, steps, *x.at++);
   float weights[SPX_LOSS_STEPS_MAX];
   for (int64_t k = 0; k < steps; ++k) weights[k] = (float)x.number();
   Unlocked released;
-  const int64_t T = mask.numel();
   const Tensor i = at::empty({LossSteps::ints(T, steps)}, mask.options().dtype(at::kInt).requires_grad(false)),
-               f = at::empty({LossSteps::floats_of(T, steps)}, mask.options().dtype(at::kFloat).requires_grad(false));
-  const LossSteps s(i, f, T, steps);
+               f = at::empty({s.all_floats()}, mask.options().dtype(at::kFloat).requires_grad(false));
+  s.bind(i, f);
   check(spx_loss_steps_mask(mask.const_data_ptr(), kind, T, (int32_t)steps, weights, s.row_map, s.live, s.inv, s.mask_sum,
                             s.full, s.ticket, stream_of(mask)),
         "spx_loss_steps_mask");
@@ -493,14 +508,16 @@ PyObject* spx_layer_loss_steps_begin(PyObject*, PyObject* const* args, Py_ssize_
   END_HANDLE_TH_ERRORS
 }
 
-// (op, mask, its kind, targets or None, their arg-max or None, integers, floats, tokens [steps, T], hits [steps, T], packed
+// (op, term weights or None, masked rows of step 0 formed?, mask, its kind, targets or None, their arg-max or None, integers, floats, tokens [steps, T], hits [steps, T], packed
 // gradient [steps * T, vocab] or None, steps, first step, logits [T, vocab] of this and the following steps ..)
 PyObject* spx_layer_loss_steps_pass(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  const int64_t here = n - 12;
+  const int64_t here = n - 14;
   TORCH_CHECK_TYPE(here >= 1 && here <= SPX_LOSS_STEPS_MAX, "loss_steps_pass takes the logits of 1 .. 32 steps");
   Args x("loss_steps_pass", args, n, n);
   const int64_t op = x.integer();
+  PyObject* const term_weights = *x.at++;
+  const int64_t masked_first = x.integer();
   const Tensor& mask = x.tensor();
   const int64_t kind = x.integer();
   const Tensor y = x.maybe(), known = x.maybe();
@@ -525,11 +542,12 @@ PyObject* spx_layer_loss_steps_pass(PyObject*, PyObject* const* args, Py_ssize_t
                         (!packed.defined() || (packed.numel() == steps * T * vocab && packed.is_contiguous() &&
                                                packed.scalar_type() == at::kBFloat16)),
                     "targets, their arg-max, tokens, hits or gradient do not fit the logits");
+  LossSteps s(T, steps, term_weights);
+  s.bind(i, f);
   Unlocked released;
-  const LossSteps s(i, f, T, steps);
-  check(spx_loss_steps_pass((int)op, logits, ld, y.defined() ? in(y) : nullptr, y.defined() ? y.stride(0) : 0,
+  check(spx_loss_steps_pass((int)op, s.terms, s.weights, logits, ld, y.defined() ? in(y) : nullptr, y.defined() ? y.stride(0) : 0,
                             known.defined() ? known.const_data_ptr<int32_t>() : nullptr, T, vocab, (int32_t)steps,
-                            (int32_t)first, (int32_t)(first + here), mask.const_data_ptr(), kind, s.inv, s.row_map, s.live,
+                            (int32_t)first, (int32_t)(first + here), masked_first != 0, mask.const_data_ptr(), kind, s.inv, s.row_map, s.live,
                             s.loss, tokens.mutable_data_ptr<int64_t>(), hits.mutable_data_ptr<uint8_t>(), s.row_slot,
                             s.slot_row, s.slots, s.row_weight, packed.defined() ? to(packed) : nullptr, vocab,
                             stream_of(mask)),
@@ -539,10 +557,12 @@ PyObject* spx_layer_loss_steps_pass(PyObject*, PyObject* const* args, Py_ssize_t
   END_HANDLE_TH_ERRORS
 }
 
-// (mask, its kind, prev or None, its kind, integers, floats, hits, steps, term factor) -> (scalars [steps, 8], loss)
+// (term weights or None, mask, its kind, prev or None, its kind, integers, floats, hits, steps, term factor) -> (scalars
+// [steps, 8], of several terms [steps, 18], loss)
 PyObject* spx_layer_loss_steps_end(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Args x("loss_steps_end", args, n, 9);
+  Args x("loss_steps_end", args, n, 10);
+  PyObject* const term_weights = *x.at++;
   const Tensor& mask = x.tensor();
   const int64_t kind = x.integer();
   const Tensor prev = x.maybe();
@@ -553,12 +573,13 @@ PyObject* spx_layer_loss_steps_end(PyObject*, PyObject* const* args, Py_ssize_t 
   const int64_t T = mask.numel();
   TORCH_CHECK_VALUE(hits.numel() == steps * T && (!prev.defined() || (prev.numel() >= T && prev.is_contiguous())),
                     "hits or prev do not fit the mask");
+  LossSteps s(T, steps, term_weights);
+  s.bind(i, f);
   Unlocked released;
-  const LossSteps s(i, f, T, steps);
-  const Tensor out = at::empty({steps, 8}, f.options()), total = at::empty({}, f.options());
+  const Tensor out = at::empty({steps, s.terms ? 18 : 8}, f.options()), total = at::empty({}, f.options());
   check(spx_loss_steps_total(s.loss, hits.const_data_ptr<uint8_t>(), mask.const_data_ptr(), kind,
                              prev.defined() ? prev.mutable_data_ptr() : nullptr, prev_kind, T, (int32_t)steps, (float)factor,
-                             s.inv, s.mask_sum, s.full, s.partials, s.ticket, floats(out), floats(total), stream_of(mask)),
+                             s.terms, s.weights, s.inv, s.mask_sum, s.full, s.partials, s.ticket, floats(out), floats(total), stream_of(mask)),
         "spx_loss_steps_total");
   return tuple_of(released, {out, total});
   END_HANDLE_TH_ERRORS

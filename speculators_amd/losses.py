@@ -528,19 +528,19 @@ class _HeadStepsLoss(torch.autograd.Function):
         native = _lib.native()
         kind = _lib.kind_code(run.mask)
         grad = run.grad
-        ints, floats, count, row_slot, slot_row, row_weight = native.loss_steps_begin(run.mask, kind, *run.weights)
+        ints, floats, count, row_slot, slot_row, row_weight = native.loss_steps_begin(run.mask, kind, run.terms, *run.weights)
         run.tokens = torch.empty(steps, t, device=dev, dtype=torch.int64)
         hits = torch.empty(steps, t, device=dev, dtype=torch.uint8)
         packed = torch.empty(steps * t, vocab, device=dev, dtype=torch.bfloat16) if grad else None
         at_once = max(1, STEPS_LOGITS_BYTES // (2 * t * vocab))
         for first in range(0, steps, at_once):
             logits = [matmul_nt(x.reshape(t, x.shape[-1]), weight) for x in xs[first:first + at_once]]
-            native.loss_steps_pass(run.op, run.mask, kind, run.targets, run.argmax, ints, floats, run.tokens, hits, packed, steps,
-                                   first, *logits)
+            native.loss_steps_pass(run.op, run.terms, run.masked_first, run.mask, kind, run.targets, run.argmax, ints, floats,
+                                   run.tokens, hits, packed, steps, first, *logits)
             if run.logits is not None:
                 run.logits += logits
         run.scalars, total = native.loss_steps_end(
-            run.mask, kind, run.prev, _lib.kind_code(run.prev) if run.prev is not None else 0, ints, floats, hits, steps,
+            run.terms, run.mask, kind, run.prev, _lib.kind_code(run.prev) if run.prev is not None else 0, ints, floats, hits, steps,
             run.factor)
         if grad:
             ctx.save_for_backward(packed, row_slot, count, weight_t, row_weight, slot_row)
@@ -557,10 +557,11 @@ class _HeadStepsLoss(torch.autograd.Function):
 
 @dataclass
 class HeadSteps:
-    """One loss (``op``: kl or ce) of all steps behind the frozen head: per-step ``weights`` of the masked mean, the term's
-    ``factor``, 1-D ``mask`` and ``prev`` (advanced in place), ``targets`` ``[T, vocab]`` or for ce their ``argmax``.  Filled
-    by ``head_steps_loss``: ``tokens`` int64 ``[steps, T]``, ``scalars`` f32 ``[steps, 8]`` (``spx_ttt_step_total``) and,
-    where it is a list before, ``logits``."""
+    """One loss (``op``: kl or ce) of all steps behind the frozen head, or a sum of several (``terms``: five weights by op, None
+    for those that are none): per-step ``weights`` of the masked mean, the one term's ``factor``, 1-D ``mask`` and ``prev`` (advanced in
+    place), ``targets`` ``[T, vocab]`` or for ce alone their ``argmax``; ``masked_first``: the first step's masked rows have a loss.
+    Filled by ``head_steps_loss``: ``tokens`` int64 ``[steps, T]``, ``scalars`` f32 ``[steps, 8]`` (``spx_ttt_step_total``; of
+    several terms ``[steps, 18]``, ``spx_ttt_step_terms``) and, where it is a list before, ``logits``."""
 
     op: int
     weights: list
@@ -570,25 +571,32 @@ class HeadSteps:
     targets: torch.Tensor | None
     argmax: torch.Tensor | None
     logits: list | None = None
+    terms: tuple | None = None
+    masked_first: bool = True
     grad: bool = False
     tokens: torch.Tensor | None = None
     scalars: torch.Tensor | None = None
 
 
-def steps_fit(op: int, steps: int, x, weight, targets, mask) -> bool:
-    """Whether ``head_steps_loss`` takes the steps: rows of the targets (``[T, vocab]``; None: ce by known arg-max) and
-    logits that fit a workgroup's registers, as ``_one_pass_ok``, of 4096 columns on as ``TERMS_MIN_VOCAB``.  From two
-    steps on: it has something to share."""
-    if not (HEAD_LOSS_ONE_PASS and 2 <= steps <= LOSS_STEPS_MAX and op in (OP_KL, OP_CE) and mask is not None):
+STEPS_OPS = (OP_KL, OP_CE, OP_TV)  # rkl and jsd do not fit the registers
+
+
+def steps_fit(loss_config, steps: int, x, weight, mask) -> bool:
+    """Whether ``head_steps_loss`` takes the steps: terms of ``STEPS_OPS`` and logits that fit a workgroup's registers, as
+    ``_one_pass_ok``, of 4096 columns on as ``TERMS_MIN_VOCAB``.  From two steps on: it has something to share."""
+    if not (HEAD_LOSS_ONE_PASS and 2 <= steps <= LOSS_STEPS_MAX and mask is not None):
+        return False
+    if any(PRIMITIVE_OP.get(name) not in STEPS_OPS or fn is not _HIP_LOSS_FN_MAP[name] for name, (fn, _) in loss_config.items()):
         return False
     t, vocab = mask.numel(), weight.shape[0]
-    if (t < steps or t * steps >= 1 << 31 or x.shape[:-1] != (1, t) or x.dtype != torch.bfloat16
-            or weight.dtype != torch.bfloat16 or vocab % 8 or not TERMS_MIN_VOCAB <= vocab <= 32768):
-        return False
-    if targets is None:
-        return op == OP_CE
-    return (targets.dtype == torch.bfloat16 and targets.shape == (t, vocab) and targets.stride(1) == 1
-            and targets.stride(0) % 8 == 0 and targets.data_ptr() % 16 == 0)
+    return (t >= steps and t * steps < 1 << 31 and x.shape[:-1] == (1, t) and x.dtype == weight.dtype == torch.bfloat16
+            and vocab % 8 == 0 and TERMS_MIN_VOCAB <= vocab <= 32768)
+
+
+def steps_rows_fit(rows, t: int, vocab: int) -> bool:
+    """Whether ``rows`` can be the target rows of ``head_steps_loss``."""
+    return (rows.dtype == torch.bfloat16 and rows.shape == (t, vocab) and rows.stride(1) == 1 and rows.stride(0) % 8 == 0
+            and rows.data_ptr() % 16 == 0)
 
 
 def head_steps_loss(run: HeadSteps, weight, weight_t, xs):

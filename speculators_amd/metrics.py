@@ -180,24 +180,19 @@ def _terms_step(head, targets, loss_mask, prev_correct, ttt_step, decay, loss_co
     return (total, m, am_d) if return_pred else (total, m)
 
 
-def _steps_targets(targets, op: int):
-    """``(rows [T, vocab], arg-max)`` of the verifier for ``losses.head_steps_loss``: for ce behind the lazily applied head
-    the arg-max alone."""
-    if isinstance(targets, VerifierHead):
-        if op == L.OP_CE and targets.logits is None:
-            return None, targets.stats()[1]
-        targets = targets.materialize()
-    return targets[0], None
-
-
 class TTTSteps:
     """``compute_metrics`` of all steps of a TTT loop at once, where one node takes them (``losses.head_steps_loss``):
-    a loss of one kl or ce term over bf16 rows, with a loss mask.  ``add`` a step's head input, ``finish`` behind the last."""
+    terms of kl, ce and tv over bf16 rows, with a loss mask.  ``add`` a step's head input, ``finish`` behind the last."""
 
-    def __init__(self, op, steps, targets, loss_mask, prev_correct, decay, factor):
-        self.op, self.steps, self.targets = op, steps, targets
-        self.mask, self.prev, self.factor = loss_mask, prev_correct, factor
+    def __init__(self, config, steps, targets, loss_mask, prev_correct, decay):
+        self.config, self.steps, self.targets = config, steps, targets
+        self.mask, self.prev = loss_mask, prev_correct
         self.weights = [float(np.float32(decay) ** np.float32(k)) for k in range(steps)]
+        ops = {L.PRIMITIVE_OP[name]: float(w) for name, (_, w) in config.items()}
+        self.op = next(iter(ops))
+        self.factor = ops[self.op]
+        # one kl or ce has a form of its own
+        self.terms = None if len(ops) == 1 and self.op != L.OP_TV else tuple(ops.get(op) for op in range(5))
         self.xs = []
 
     @staticmethod
@@ -205,36 +200,36 @@ class TTTSteps:
         """The steps behind ``x`` (the first one's head input), or None where ``compute_metrics`` has to take them."""
         if loss_config is None:
             loss_config = {"kl_div": (L.kl_div_loss, 1.0)}
-        if (compute_metrics is not _own_compute_metrics or len(loss_config) != 1 or loss_mask is None
-                or isinstance(targets, TargetGather)):
+        if (compute_metrics is not _own_compute_metrics or loss_mask is None or not loss_config
+                or not L.steps_fit(loss_config, steps, x, weight, loss_mask)):
             return None
-        (name, (fn, factor)), = loss_config.items()
-        op = L.PRIMITIVE_OP.get(name)
-        if op not in (L.OP_KL, L.OP_CE) or fn is not L._HIP_LOSS_FN_MAP[name]:
+        shape, vocab = tuple(x.shape[:-1]), weight.shape[0]
+        if tuple(loss_mask.shape) != shape or tuple(prev_correct.shape) != shape:
             return None
-        shape = tuple(x.shape[:-1])
-        if shape[0] != 1 or tuple(loss_mask.shape) != shape or tuple(prev_correct.shape) != shape:
-            return None
-        rows = None
         if isinstance(targets, VerifierHead):  # (its rows are bf16, contiguous, of its weight's width)
-            fits = targets.x.shape[1] == shape[1] and targets.weight.shape[0] == weight.shape[0]
-            op_rows = L.steps_fit(L.OP_CE, steps, x, weight, None, loss_mask)
-            if not (fits and op_rows and targets.weight.dtype == torch.bfloat16):
-                return None
+            fits = targets.x.shape[1] == shape[1] and targets.weight.shape[0] == vocab and targets.weight.dtype == torch.bfloat16
+        elif isinstance(targets, TargetGather):
+            fits = (targets.full.shape[:2] == shape and targets.full.dtype == torch.bfloat16 and targets.d2t.numel() == vocab
+                    and targets.compact is None)
         else:
-            rows = targets[0] if targets.dim() == 3 and targets.shape[0] == 1 else None
-            if rows is None or not L.steps_fit(op, steps, x, weight, rows, loss_mask):
-                return None
-        return TTTSteps(op, steps, targets, _as_mask(loss_mask), _flat_prev(prev_correct), decay, float(factor))
+            fits = targets.dim() == 3 and targets.shape[0] == 1 and L.steps_rows_fit(targets[0], shape[1], vocab)
+        return TTTSteps(loss_config, steps, targets, _as_mask(loss_mask), _flat_prev(prev_correct), decay) if fits else None
 
     def add(self, x):
         self.xs.append(x)
 
     def finish(self, weight, weight_t, logits=None):
         """``(loss, metrics, draft tokens of every step [1, T])``; ``logits``: a list that receives every step's."""
-        rows, argmax = _steps_targets(self.targets, self.op)
+        rows = argmax = None
+        targets = self.targets
+        if isinstance(targets, VerifierHead) and self.terms is None and self.op == L.OP_CE and targets.logits is None:
+            argmax = targets.stats()[1]  # no target row exists
+        else:
+            rows = (targets if isinstance(targets, torch.Tensor) else targets.materialize())[0]
         kept = None if logits is None else []
-        run = L.HeadSteps(self.op, self.weights, self.factor, self.mask, self.prev, rows, argmax, kept)
+        # (the pass that gathers a first step's rows for several terms knows their statistics: masked rows are not formed)
+        run = L.HeadSteps(self.op, self.weights, self.factor if self.terms is None else 1.0, self.mask, self.prev, rows, argmax, kept,
+                          self.terms, not (self.terms and isinstance(targets, TargetGather)))
         loss = L.head_steps_loss(run, weight, weight_t, self.xs)
         if logits is not None:
             logits += [x.view(1, *x.shape) for x in kept]
@@ -242,6 +237,10 @@ class TTTSteps:
         for k in range(self.steps):
             out = run.scalars[k]
             m[f"loss_{k}_sum"], m[f"loss_{k}_total"] = out[6], out[7]
+            if len(self.config) > 1:
+                for name in self.config:
+                    op = L.PRIMITIVE_OP[name]
+                    m[f"{name}_loss_{k}_sum"], m[f"{name}_loss_{k}_total"] = out[8 + op], out[13 + op]
             m[f"full_acc_{k}_sum"], m[f"full_acc_{k}_total"] = out[1], out[2]
             m[f"cond_acc_{k}_sum"], m[f"cond_acc_{k}_total"] = out[3], out[4]
         return loss, m, list(run.tokens.split(1))

@@ -56,7 +56,8 @@ def _close(a, b, rel):
 
 # edges of a workgroup's chunks (512 x 8 columns), of the reduction's 256 rows and of the rows that have no target
 @pytest.mark.parametrize("t,steps,vocab", [(2, 2, 4096), (7, 7, 4104), (255, 3, 32000), (257, 5, 32768), (600, 32, 4160)])
-@pytest.mark.parametrize("name", ["kl_div", "ce"])
+@pytest.mark.parametrize("name", ["kl_div", "ce", "tv", '{"ce": 0.1, "tv": 0.9}', '{"kl_div": 0.5, "ce": 0.2}',
+                                  '{"tv": 1.5, "kl_div": 0.25, "ce": 0.125}'])
 def test_steps_together(t, steps, vocab, name):
     from speculators_amd import losses as L
 
@@ -121,6 +122,27 @@ def test_steps_in_several_passes_and_extreme_rows(monkeypatch):
     assert torch.equal(again[0], got[0]) and all(torch.equal(a, b) for a, b in zip(again[4], got[4], strict=True))
 
 
+@pytest.mark.parametrize("name", ["kl_div", "ce", '{"ce": 0.1, "tv": 0.9}'])
+def test_targets_gathered_from_the_full_vocabulary(name):
+    from speculators_amd import losses as L
+    from speculators_amd import metrics as MT
+
+    x, w, y, mask = _case(70, 3, 4096, 5)
+    g = torch.Generator().manual_seed(2)
+    ids = torch.randperm(9000, generator=g)[:4096].sort().values.cuda()
+    full = torch.randn(1, 70, 9000, generator=g).bfloat16().cuda()
+    full[..., ids] = y
+    d2t = ids - torch.arange(4096, device="cuda")
+    config = L.resolve_loss_config(name)
+    want = _together(x, w, y, mask, 0.9, config)
+    got = _together(x, w, MT.TargetGather(full, d2t), mask, 0.9, config)
+    assert torch.equal(got[0], want[0]) and all(torch.equal(a, b) for a, b in zip(got[2] + list(got[4]), want[2] + list(want[4])))
+    old = _one_by_one(x, w, MT.TargetGather(full, d2t), mask, 0.9, config)
+    _close(got[0], old[0], 4e-6)
+    for a, b in zip(got[4], old[4], strict=True):
+        _close(a, b, 2.0 ** -8)
+
+
 def test_what_goes_step_by_step():
     from speculators_amd import losses as L
     from speculators_amd import metrics as MT
@@ -133,6 +155,7 @@ def test_what_goes_step_by_step():
 
     assert taken() and taken(config=None)
     assert not taken(steps=1) and not taken(steps=25) and not taken(steps=33) and not taken(m=None)
-    assert not taken(config=L.resolve_loss_config("tv")) and not taken(config=L.resolve_loss_config('{"ce": 1, "kl_div": 1}'))
+    assert taken(config=L.resolve_loss_config("tv")) and not taken(config=L.resolve_loss_config('{"ce": 1, "rkl": 1}'))
+    assert not taken(config=L.resolve_loss_config("jsd")) and not taken(config=L.resolve_loss_config("nla"))
     assert not taken(config={"kl_div": (lambda a, b: a, 1.0)}) and not taken(targets=y.float())
     assert not taken(targets=y[..., 1:], weight=w[1:]) and not taken(targets=y[..., :4088], weight=w[:4088])
