@@ -192,6 +192,14 @@ int spx_label_ce_from_lse(const void* logits, int64_t ld_logits, const int64_t* 
                           int64_t rows, int64_t vocab, int dtype, int64_t ignore_index,
                           const float* lse, float* loss, void* stream);
 
+/* The loss and, for rows whose label is not the ignored one, the logits gradient for a row weight of ONE, packed to the front
+ * (bf16; vocab a multiple of 8, at most 155648): row_map [rows] = the slot of a live row or -1, row_of [rows] = the live rows in
+ * their order (slots past *count are not written), grad_logits[row_map[r], :] = softmax(logits[r, :]) - onehot(labels[r]).
+ * Followed by spx_gemm_bf16_rows_graded, which applies the weights of the rows. */
+int spx_label_ce_fwd_grad(const void* logits, int64_t ld_logits, const int64_t* labels, int64_t rows, int64_t vocab,
+                          int64_t ignore_index, float* loss, int32_t* row_map, int32_t* count, int32_t* row_of,
+                          void* grad_logits, int64_t ld_grad, void* stream);
+
 /* dlogits[r, j] = grad_rows[r] * (softmax(logits[r, :])[j] - [j == labels[r]]);
  * rows with grad_rows[r] == 0 or an ignored label are exact zeros and are not
  * read.  The autograd backward of the call above (models/mtp/core.py:204-218). */

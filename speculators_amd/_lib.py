@@ -92,6 +92,7 @@ SIGNATURES["spx_swiglu_fwd"] = [_P, _P, _P, _I64, _P]
 SIGNATURES["spx_swiglu_bwd"] = [_P, _P, _P, _P, _P, _I64, _P]
 SIGNATURES["spx_label_ce_fwd"] = [_P, _I64, _P, _I64, _I64, _I, _I64, _P, _P, _P, _P]
 SIGNATURES["spx_label_ce_from_lse"] = [_P, _I64, _P, _I64, _I64, _I, _I64, _P, _P, _P]
+SIGNATURES["spx_label_ce_fwd_grad"] = [_P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _I64, _P]
 SIGNATURES["spx_label_ce_bwd"] = [_P, _I64, _P, _P, _P, _I64, _I64, _I, _I64, _P, _I64, _P]
 SIGNATURES["spx_label_ce_bwd_packed"] = [_P, _I64, _P, _P, _P, _I64, _I64, _I, _I64, _P, _P, _I64, _P]
 SIGNATURES["spx_pack_batch"] = [_P, _I, _I64, _I64, _I64, _P, _P, _I, _P, _P, _P, _I64, _I64, _I,

@@ -8,7 +8,6 @@
 // pre-scaled by log2(e), statistics are converted back at the end.
 
 #include <algorithm>
-#include <type_traits>
 
 #include "loss_common.h"
 #include "../../include/spx.h"
@@ -1254,27 +1253,6 @@ __global__ __launch_bounds__(1024) void mask_row_map_kernel(const void* __restri
                                                             int32_t* __restrict__ row_of, int32_t* __restrict__ zero3) {
   if (zero3 && threadIdx.x < 3) zero3[threadIdx.x] = 0;
   pack_row_map([&](int r) { return mask_value(mask, mask_kind, r) != 0.f; }, rows, row_map, count, row_of);
-}
-
-// op over the 64 lanes, every lane gets the result: moves inside the sixteen lanes of a row, then swaps of rows, where a
-// shuffle would be a trip through LDS (six of them a value: kl, 4096 rows x 7 steps 748 -> 719 us)
-template <typename T, typename Op>
-__device__ __forceinline__ T wave_all(T v, Op op) {
-  static_assert(sizeof(T) == 4, "one register");
-  auto moved = [](T x, auto ctrl) __attribute__((always_inline)) {
-    const int i = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xf, 0xf, true));
-  };
-  v = op(v, moved(v, std::integral_constant<int, 0xb1>{}));   // quad_perm 1 0 3 2
-  v = op(v, moved(v, std::integral_constant<int, 0x4e>{}));   // quad_perm 2 3 0 1
-  v = op(v, moved(v, std::integral_constant<int, 0x141>{}));  // row_half_mirror
-  v = op(v, moved(v, std::integral_constant<int, 0x140>{}));  // row_mirror
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = op(__builtin_bit_cast(T, (uint32_t)rows[0]), __builtin_bit_cast(T, (uint32_t)rows[1]));
-  u = __builtin_bit_cast(uint32_t, v);
-  const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return op(__builtin_bit_cast(T, (uint32_t)halves[0]), __builtin_bit_cast(T, (uint32_t)halves[1]));
 }
 
 // ---- all steps of a TTT loop at one target row -------------------------------------------------------

@@ -180,6 +180,118 @@ __global__ __launch_bounds__(256) void label_ce_pick_kernel(const T* __restrict_
   loss[r] = l;
 }
 
+// ---- forward and logits gradient in one read -------------------------------------------------------
+// Rows that carry a gradient are known before the loss is (labels), and the gradient but for the weight of its row: one
+// workgroup of 1024 threads holds a whole row of up to 155648 columns in registers (19 chunks of 16 bytes a thread), reduces
+// it, and goes over the registers a second time for softmax(x) - onehot(label), the gradient of a row of weight ONE, packed to
+// the front; the input-gradient product, which is linear in it, applies the weights (spx_gemm_bf16_rows_graded).  A
+// workgroup walks its rows, and behind every stored chunk it requests that chunk of its next row: loads and stores of two
+// rows are under way while one is reduced.  22930 live of 32760 rows of 151936, us: a forward and a backward pass (two
+// reads and a write) 3773, so 2725 (5.15 TB/s); 1400 of 1997 267 / 176, 350 of 510 78 / 53; 1400 of 2000 rows of 65536 112 / 78.
+constexpr int kOneThreads = 1024, kOneWaves = kOneThreads / 64, kOneChunks = 19;
+
+// row_map and row_of (the live rows in their order), and a loss of zero for the others
+__global__ __launch_bounds__(1024) void label_rows_kernel(const int64_t* __restrict__ labels, int64_t ignore_index, int rows,
+                                                          int32_t* __restrict__ row_map, int32_t* __restrict__ count,
+                                                          int32_t* __restrict__ row_of, float* __restrict__ loss) {
+  pack_row_map([&](int r) {
+    const bool live = labels[r] != ignore_index;
+    if (!live) loss[r] = 0.f;
+    return live;
+  }, rows, row_map, count, row_of);
+}
+
+__global__ __launch_bounds__(kOneThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void label_ce_fwd_grad_kernel(
+    const uint16_t* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels, int vocab,
+    const int32_t* __restrict__ row_of, const int32_t* __restrict__ count, float* __restrict__ loss,
+    uint16_t* __restrict__ grad, int64_t ld_grad) {
+  __shared__ float sm[2][kOneWaves], sz[2][kOneWaves];
+  const int n = *count, tid = threadIdx.x, nchunks = vocab >> 3;
+  int slot = blockIdx.x;
+  if (slot >= n) return;
+  int r = row_of[slot];
+  const uint16_t* row = logits + (int64_t)r * ld;
+  u32x4 xr[kOneChunks];
+#pragma unroll
+  for (int j = 0; j < kOneChunks; ++j) {
+    const int c = tid + j * kOneThreads;
+    if (c < nchunks) xr[j] = ld16(row + ((int64_t)c << 3));
+  }
+  auto unpack = [](u32x4 raw, float (&v)[8]) __attribute__((always_inline)) {
+    v[0] = bf16_lo(raw.x); v[1] = bf16_hi(raw.x); v[2] = bf16_lo(raw.y); v[3] = bf16_hi(raw.y);
+    v[4] = bf16_lo(raw.z); v[5] = bf16_hi(raw.z); v[6] = bf16_lo(raw.w); v[7] = bf16_hi(raw.w);
+  };
+  for (int turn = 0;; turn ^= 1) {
+    const int64_t label = labels[r];
+    const bool inside = label >= 0 && label < vocab;
+    const float xt = tid == 0 && inside ? load1(row + label) : __builtin_nanf("");
+    const int next = slot + (int)gridDim.x;
+    const bool more = next < n;
+    const int nr = more ? row_of[next] : 0;
+    // (places of chunks worked out where they are needed: kept over the rows they would be spilled, and a reload waits for
+    // every load in front of it)
+    int lane0 = tid;
+    asm volatile("" : "+v"(lane0));
+    float m = kNegBig, z = 0.f;
+#pragma unroll
+    for (int j = 0; j < kOneChunks; ++j) {
+      if (lane0 + j * kOneThreads >= nchunks) continue;
+      float x[8];
+      unpack(xr[j], x);
+      float cx = x[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) cx = fmaxf(cx, x[i]);
+      const float cs = cx * kLog2e;
+      if (cs > m) {  // the running maximum moved: rescale the sum
+        z *= fast_exp2(m - cs);
+        m = cs;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -m));
+    }
+    const float wm = wave_all(m, [](float a, float b) { return fmaxf(a, b); });
+    z = wave_all(z * fast_exp2(m - wm), [](float a, float b) { return a + b; });
+    if ((tid & 63) == 0) { sm[turn][tid >> 6] = wm; sz[turn][tid >> 6] = z; }
+    __syncthreads();
+    m = sm[turn][0];
+#pragma unroll
+    for (int w = 1; w < kOneWaves; ++w) m = fmaxf(m, sm[turn][w]);
+    z = 0.f;
+#pragma unroll
+    for (int w = 0; w < kOneWaves; ++w) z += sz[turn][w] * fast_exp2(sm[turn][w] - m);
+    const float l2 = m + fast_log2(z);
+    // (a label outside [0, vocab) that is not the ignore index has no defined loss)
+    if (tid == 0) loss[r] = l2 * kLn2 - xt;
+    uint16_t* const out = grad + (int64_t)slot * ld_grad;
+    const uint16_t* const nrow = logits + (int64_t)nr * ld;
+    asm volatile("" : "+v"(lane0));
+#pragma unroll
+    for (int j = 0; j < kOneChunks; ++j)  // (the packed chunks are what stays in registers between the passes)
+      asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
+#pragma unroll
+    for (int j = 0; j < kOneChunks; ++j) {
+      const int c = lane0 + j * kOneThreads;
+      if (c >= nchunks) continue;
+      const uint32_t base = (uint32_t)c << 3;
+      float x[8], d[8];
+      unpack(xr[j], x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d[i] = fast_exp2(fmaf(x[i], kLog2e, -l2));
+      if (inside && c == (int)(label >> 3)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d[i] -= i == (int)(label & 7) ? 1.f : 0.f;
+      }
+      store8_vec<uint16_t>(out + base, d);
+      if (more) xr[j] = ld16(nrow + base);
+      __builtin_amdgcn_sched_barrier(0);  // (one chunk's unpacked values at a time)
+    }
+    if (!more) return;
+    slot = next;
+    r = nr;
+    row = nrow;
+  }
+}
+
 }  // namespace spx
 
 using namespace spx;
@@ -273,4 +385,23 @@ extern "C" int spx_label_ce_bwd_packed(const void* logits, int64_t ld_logits, co
   if (!row_map) return fail_arg(__func__, "null row map");
   return label_ce_bwd_impl(__func__, logits, ld_logits, labels, lse, grad_rows, rows, vocab, dtype,
                            ignore_index, dlogits, ld_out, row_map, stream);
+}
+
+extern "C" int spx_label_ce_fwd_grad(const void* logits, int64_t ld_logits, const int64_t* labels, int64_t rows, int64_t vocab,
+                                     int64_t ignore_index, float* loss, int32_t* row_map, int32_t* count, int32_t* row_of,
+                                     void* grad_logits, int64_t ld_grad, void* stream) {
+  if (int rc = label_ce_checks(__func__, logits, ld_logits, labels, rows, vocab, SPX_DTYPE_BF16)) return rc;
+  SPX_REQUIRE(vocab % 8 == 0 && vocab <= (int64_t)kOneThreads * kOneChunks * 8, "vocab must be a multiple of 8, at most 155648");
+  SPX_REQUIRE(loss && row_map && count && row_of && grad_logits, "null output");
+  SPX_REQUIRE(ld_grad >= vocab && ld_grad % 8 == 0 && ld_logits % 8 == 0 && ptr_aligned16(logits) && ptr_aligned16(grad_logits),
+              "rows must be 16-byte aligned, strides at least vocab");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(label_rows_kernel, dim3(1), dim3(1024), 0, st, labels, ignore_index, (int)rows, row_map, count, row_of,
+                     loss);
+  if (int rc = check_launch(__func__)) return rc;
+  // a workgroup fills a compute unit
+  hipLaunchKernelGGL(label_ce_fwd_grad_kernel, dim3((unsigned)(rows < 256 ? rows : 256)), dim3(kOneThreads), 0, st,
+                     reinterpret_cast<const uint16_t*>(logits), ld_logits, labels, (int)vocab, row_of, count, loss,
+                     reinterpret_cast<uint16_t*>(grad_logits), ld_grad);
+  return check_launch(__func__);
 }

@@ -32,7 +32,8 @@ if not 1 <= SPLIT_PARTS <= 8:
 
 
 # parts the last round's tiles of such a product with graded rows may be cut into, and partial tiles of 256 KB held for them
-LIVE_TAIL_PARTS, LIVE_TAIL_TILES = 8, 1024
+# (22930 live rows x 151936 -> 2048: 208 tiles of a last round in 6 parts; with room for 1024 in one piece, 0.4 ms more of 10)
+LIVE_TAIL_PARTS, LIVE_TAIL_TILES = 8, 1280
 # parts the tiles of a mostly empty last round of a product may be cut into (spx_gemm_bf16_nt_tail); 1 = never
 TAIL_PARTS = int(os.environ.get("SPX_GEMM_TAIL_PARTS", "4"))
 if not 1 <= TAIL_PARTS <= 8:

@@ -785,9 +785,25 @@ class _HeadLabelCE(torch.autograd.Function):
     no gradient of their own."""
 
     @staticmethod
-    def forward(ctx, x2, weight, weight_t, labels, ignore_index, epilogue_stats=False):
+    def forward(ctx, x2, weight, weight_t, labels, ignore_index, epilogue_stats=False, one_pass=False):
         from .gemm import gemm_nt_stats, matmul_nt
 
+        ctx.one_pass = False
+        if one_pass and not epilogue_stats:
+            logits = matmul_nt(x2, weight)
+            packed = _room_for_gradient(logits)
+            if packed is not None:
+                ctx.one_pass = True
+                rows, vocab = logits.shape
+                loss = torch.empty(rows, device=logits.device, dtype=torch.float32)
+                lists = torch.empty(2 * rows + 1, device=logits.device, dtype=torch.int32)
+                row_map, row_of, count = lists[:rows], lists[rows:2 * rows], lists[2 * rows:]
+                _lib.call("spx_label_ce_fwd_grad", logits, logits.stride(0), labels, rows, vocab, int(ignore_index), loss,
+                          row_map, count, row_of, packed, vocab, _lib.stream_ptr(logits.device))
+                ctx.save_for_backward(packed, row_map, count, weight_t, row_of)
+                ctx.mark_non_differentiable(logits)
+                ctx.set_materialize_grads(False)
+                return loss, logits
         if epilogue_stats:
             # the head product's epilogue leaves every row's log-sum-exp; the loss then reads one
             # element of each row instead of streaming the [rows, V] logits a second time
@@ -799,7 +815,8 @@ class _HeadLabelCE(torch.autograd.Function):
                       vocab, _lib.dtype_code(logits), int(ignore_index), out[1], out[0],
                       _lib.stream_ptr(logits.device))
         else:
-            logits = matmul_nt(x2, weight)
+            if not one_pass:
+                logits = matmul_nt(x2, weight)
             rows, vocab = logits.shape
             out = torch.empty(2, rows, device=logits.device, dtype=torch.float32)
             _lib.call("spx_label_ce_fwd", logits, logits.stride(0), labels, rows,
@@ -813,10 +830,18 @@ class _HeadLabelCE(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_rows, _grad_logits):
-        from .gemm import matmul_nt
+        from .gemm import matmul_nt, rows_graded
 
         if grad_rows is None:
-            return (None,) * 6
+            return (None,) * 7
+        if ctx.one_pass:
+            packed, row_map, count, weight_t, row_of = ctx.saved_tensors
+            g = grad_rows.to(torch.float32).contiguous()
+            one = torch.ones((), device=g.device, dtype=torch.float32)
+            dx = rows_graded(packed, weight_t, count, row_of, g, one, 1.0)
+            # (a row whose incoming gradient is zero has a gradient of zero, whatever its logits are)
+            dx = _unpack_rows(dx, torch.where(g == 0, -1, row_map), row_map.numel())
+            return (dx,) + (None,) * 6
 
         logits, labels, lse, weight_t = ctx.saved_tensors
         rows, vocab = logits.shape
@@ -828,7 +853,30 @@ class _HeadLabelCE(torch.autograd.Function):
                   row_map, packed, packed.stride(0),
                   _lib.stream_ptr(logits.device))
         dx_packed = matmul_nt(packed, weight_t, m_live=count)
-        return _unpack_rows(dx_packed, row_map, rows), None, None, None, None, None
+        return (_unpack_rows(dx_packed, row_map, rows),) + (None,) * 6
+
+
+def _label_one_pass(x2, weight, weight_t) -> bool:
+    """Whether the row pass of the frozen-head cross-entropy leaves the logits gradient behind
+    (``spx_label_ce_fwd_grad``): rows that fit a workgroup's registers and give every thread eight chunks at least."""
+    vocab = weight.shape[0]
+    return (HEAD_LOSS_ONE_PASS and torch.is_grad_enabled() and x2.requires_grad and vocab % 8 == 0 and 65536 <= vocab <= 155648
+            and 0 < x2.shape[0] < 1 << 31)
+
+
+# of the card's memory, what one call's gradient may take from its forward to its backward
+LABEL_GRADIENT_SHARE = 1 / 24
+
+
+def _room_for_gradient(logits):
+    """Where the logits gradient waits for the backward, or None: it is made there then, from the logits."""
+    total = torch.cuda.get_device_properties(logits.device).total_memory
+    if logits.numel() * 2 > total * LABEL_GRADIENT_SHARE:
+        return None
+    try:
+        return torch.empty_like(logits)
+    except torch.OutOfMemoryError:
+        return None
 
 
 # Whether the frozen-head cross-entropy takes its row statistics from the head product's epilogue
@@ -858,7 +906,8 @@ def head_label_cross_entropy(x: torch.Tensor, weight: torch.Tensor, weight_t: to
     lab = labels.reshape(-1).to(torch.int64).contiguous()
     if epilogue_stats is None:
         epilogue_stats = HEAD_CE_EPILOGUE_STATS
-    loss, logits = _HeadLabelCE.apply(x2, weight, weight_t, lab, ignore_index, bool(epilogue_stats))
+    loss, logits = _HeadLabelCE.apply(x2, weight, weight_t, lab, ignore_index, bool(epilogue_stats),
+                                      _label_one_pass(x2, weight, weight_t))
     return loss.view(labels.shape), logits.view(*labels.shape, weight.shape[0])
 
 
