@@ -257,7 +257,7 @@ def kernel_rooflines(torch, cfg, t, k_steps, device, windows=(None,)):
     from speculators_amd import _lib
     from speculators_amd import attention as A
     from speculators_amd import losses as L
-    from speculators_amd.gemm import gemm_nt, gemm_tn
+    from speculators_amd.gemm import gemm_nt, gemm_tn, rows_graded
     from speculators_amd.data import plan_rows
 
     h, vd = cfg["hidden_size"], cfg["draft_vocab_size"]
@@ -315,7 +315,7 @@ def kernel_rooflines(torch, cfg, t, k_steps, device, windows=(None,)):
     wt = w.t().contiguous()
     dx = torch.empty(t, h, device=device, dtype=torch.bfloat16)
     ms = time_events(torch, lambda: gemm_nt(y, wt, dx), 20)
-    mfma("gemm_bf16_nt_kernel[lm_head dX T x Vd x H]", 2.0 * t * h * vd, ms, k_steps, "gemm_dx")
+    mfma("gemm_bf16_nt_kernel[lm_head dX T x Vd x H]", 2.0 * t * h * vd, ms, 0, "gemm_dx")
     del wt, dx
 
     # fused loss forward / backward over T rows (step 0 shape)
@@ -368,7 +368,7 @@ def kernel_rooflines(torch, cfg, t, k_steps, device, windows=(None,)):
 
     ms = time_events(torch, loss_bwd_packed, 20)
     hbm(f"loss_bwd_kernel[KL, packed: {n_live} live of T rows x Vd]", 3.0 * n_live * vd * 2, ms, 0)
-    # what the timed step launches while lm_head is frozen: loss, statistics, acceptance chain AND the
+    # one step's row pass while lm_head is frozen: loss, statistics, acceptance chain AND the
     # unit-weight logits gradient of the live rows in one read of the row pair.  Step 0 reads every target row
     # (their statistics are made there), the later steps only those of the live rows.
     mask_f = live_mask.float()
@@ -379,11 +379,29 @@ def kernel_rooflines(torch, cfg, t, k_steps, device, windows=(None,)):
     known_fg = (fg0[1].clone(), fg0[3].clone())
     ms = time_events(torch, lambda: L._loss_forward_with_grad(L.OP_KL, lg, tg, None, step_fg), 20)
     hbm(f"loss_fwd_grad_kernel[KL forward + logits gradient of {n_live} live rows, step 0, + row map]",
-        (2.0 * t + n_live) * vd * 2, ms, 1, "loss_fwd_grad_step0")
+        (2.0 * t + n_live) * vd * 2, ms, 0, "loss_fwd_grad_step0")
     ms = time_events(torch, lambda: L._loss_forward_with_grad(L.OP_KL, lg, tg, known_fg, step_fg), 20)
     hbm(f"loss_fwd_grad_kernel[KL forward + logits gradient of {n_live} live rows, steps >= 1, + row map]",
-        (1.0 * t + 2.0 * n_live) * vd * 2, ms, k_steps - 1, "loss_fwd_grad")
+        (1.0 * t + 2.0 * n_live) * vd * 2, ms, 0, "loss_fwd_grad")
     del fg0
+    # what the timed step launches: the row pass of all steps (a target row read once for all of them), and the input gradient
+    # of the live rows of all steps as one product
+    native, kind = _lib.native(), _lib.kind_code(mask_f)
+    all_lg = [lg] + [torch.randn(t, vd, device=device, generator=g).bfloat16() for _ in range(k_steps - 1)]
+    ints, floats, count, _, slot_row, row_weight = native.loss_steps_begin(mask_f, kind, None, *([1.0] * k_steps))
+    tokens = torch.empty(k_steps, t, device=device, dtype=torch.int64)
+    hits = torch.empty(k_steps, t, device=device, dtype=torch.uint8)
+    packed = torch.empty(k_steps * t, vd, device=device, dtype=torch.bfloat16)
+    ms = time_events(torch, lambda: native.loss_steps_pass(L.OP_KL, None, 1, mask_f, kind, tg, None, ints, floats, tokens, hits,
+                                                           packed, k_steps, 0, *all_lg), 10)
+    hbm(f"loss_steps_kernel[KL, {k_steps} steps of T rows x Vd, logits gradient of {n_live} live targets]",
+        ((k_steps + 1.0) * t + k_steps * n_live) * vd * 2, ms, 1)
+    del all_lg
+    wt_all = (torch.randn(h, vd, device=device, generator=g) * 0.02).bfloat16()
+    one = torch.ones((), device=device)
+    ms = time_events(torch, lambda: rows_graded(packed, wt_all, count, slot_row, row_weight, one, 1.0), 5)
+    mfma("gemm_bf16_nt_kernel[lm_head dX, live rows of all steps x Vd x H]", 2.0 * k_steps * n_live * h * vd, ms, 1)
+    del packed, wt_all
     # the yardstick of that launch's size: a plain copy of n_live rows (one read + one write per element;
     # the kernel above reads two rows for every row it writes)
     src = lg[:n_live]
@@ -691,7 +709,18 @@ def run_mtp(args):
     lg = logits.detach().requires_grad_(True)
     out = label_cross_entropy(lg, lab)
     rec("label_ce_fwd_kernel[rows x V, 70% live rows]", "hbm", live * v * 2.0,
-        time_events(torch, lambda: label_cross_entropy(logits, lab), 5), 0 if epi_default else k_steps)
+        time_events(torch, lambda: label_cross_entropy(logits, lab), 5), 0)
+    # loss and unit-weight logits gradient in one read of the live rows: what the model launches
+    lists = torch.empty(2 * rows + 1, device=device, dtype=torch.int32)
+    unit, losses_buf = torch.empty_like(logits), torch.empty(rows, device=device)
+
+    def ce_one_read():
+        _lib.call("spx_label_ce_fwd_grad", logits, logits.stride(0), lab, rows, v, -100, losses_buf, lists[:rows], lists[2 * rows:],
+                  lists[rows:2 * rows], unit, v, _lib.stream_ptr(device))
+
+    rec("label_ce_fwd_grad_kernel[rows x V, 70% live rows, loss + logits gradient]", "hbm", 2 * live * v * 2.0,
+        time_events(torch, ce_one_read, 5), 0 if epi_default else k_steps)
+    del unit
     # the head product with every row's log-sum-exp out of its epilogue + one element per row for the loss:
     # what replaces the two launches above in the model
     lse_buf = torch.empty(rows, device=device)
@@ -716,7 +745,7 @@ def run_mtp(args):
 
     # live rows: one read + one write; dead rows: one write of zeros
     rec("label_ce_bwd_kernel[rows x V, 70% live rows]", "hbm", (2 * live + (rows - live)) * v * 2.0,
-        time_events(torch, ce_bwd, 5), k_steps)
+        time_events(torch, ce_bwd, 5), k_steps if epi_default else 0)
     dl = lg.grad
     del lg, out
     wt = w.detach().t().contiguous()
