@@ -631,6 +631,32 @@ int spx_head_norm_rope_bwd(const void* tok, int64_t ld_tok, const void* dout, in
                            int64_t ld_dtok, float* dw_scratch, int32_t accumulate, int64_t T, int32_t n_heads,
                            int32_t n_pass, int32_t D, int64_t position_offset, float table_scale, void* stream);
 
+/* Both for one or two sets of heads (a layer's queries, and its keys with the values) in one launch: every set as in the calls
+ * above (out and pass are read by the backward; eps is the forward's, the last four members the backward's).  `sets` is host
+ * memory, read before the call returns. */
+typedef struct {
+  const void* tok;
+  int64_t ld_tok;
+  void* out;
+  int64_t out_head_stride;
+  void* pass;
+  int64_t pass_head_stride;
+  const int64_t* position_ids;
+  const void* gain;
+  float* rstd;
+  int64_t T;
+  int32_t n_heads, n_pass;
+  float eps;
+  int32_t accumulate;
+  void* dtok;
+  int64_t ld_dtok;
+  float* dw_scratch;
+} spx_head_norm;
+int spx_head_norm_rope_sets(const spx_head_norm* sets, int32_t count, const float* inv_freq, int32_t D,
+                            int64_t position_offset, float table_scale, void* stream);
+int spx_head_norm_rope_bwd_sets(const spx_head_norm* sets, int32_t count, const float* inv_freq, int32_t D,
+                                int64_t position_offset, float table_scale, void* stream);
+
 /* Rotary embedding fused with the head-major relayout that precedes attention
  * (apply_rotary_pos_emb + the view/transpose of LlamaAttention.forward; for
  * DFlash models/dflash/model_definitions.py:29-45):

@@ -78,6 +78,8 @@ SIGNATURES["spx_cat_bf16"] = [_P, _P, _P, _I32, _P, _P]
 SIGNATURES["spx_head_norm_rope"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I64, _F, _F, _P]
 SIGNATURES["spx_head_norm_rope_bwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I32, _I64, _I32, _I32,
                                         _I32, _I64, _F, _P]
+SIGNATURES["spx_head_norm_rope_sets"] = [_P, _I32, _P, _I32, _I64, _F, _P]
+SIGNATURES["spx_head_norm_rope_bwd_sets"] = [_P, _I32, _P, _I32, _I64, _F, _P]
 SIGNATURES["spx_rmsnorm_bwd_slots"] = [_I64, _I64]
 SIGNATURES["spx_rmsnorm_bwd"] = [_P, _I64, _P, _P, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _P]
 SIGNATURES["spx_add_rmsnorm_fwd"] = [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P, _I64, _I64, _F, _P]

@@ -451,19 +451,30 @@ __global__ __launch_bounds__(256) void rope_qkv_kernel(uint16_t* __restrict__ to
 // separate kernels: bf16(x * rstd), its product with the gain, each product and the sum of the rotation.  D / 16 lanes share
 // a head, each with the two chunks of eight that rotate together; a thread works on HEADS heads of one token and evaluates
 // the angles once.  Bound by HBM where the rows fill the chip; one read and one write of q and k where the norm and the
-// relayout made two each (16384 tokens, 16 + 2 heads of 256: 345 us -> 91, the way back 375 -> 120).
+// relayout made two each (16384 tokens, 16 + 2 heads of 256: 345 us -> 91, the way back 375 -> 120).  A layer's queries and its
+// keys with the values go in one launch: workgroups from `first` on have the second set (three layers of 888 / 2665
+// rows of 32 and 8 + 8 heads of 64, forward 42 -> 28 us, back 49 -> 39; five of 8192 / 16384 of 128 378 -> 351, 530 -> 484).
+struct HeadSets {
+  spx_head_norm set[2];
+  int first;      // workgroups of set 0
+};
 template <int D, int HEADS>
-__global__ __launch_bounds__(256) void head_norm_rope_kernel(const uint16_t* __restrict__ tok, int64_t ld,
-                                                             uint16_t* __restrict__ out, int64_t hs_out,
-                                                             uint16_t* __restrict__ pass, int64_t hs_pass,
-                                                             const int64_t* __restrict__ pos,
-                                                             const float* __restrict__ inv_freq,
-                                                             const uint16_t* __restrict__ gain, float* __restrict__ rstd,
-                                                             int T, int n_heads, int n_pass, int64_t pos_offset,
-                                                             float table_scale, float eps) {
+__global__ __launch_bounds__(256) void head_norm_rope_kernel(HeadSets sets, const float* __restrict__ inv_freq,
+                                                             int64_t pos_offset, float table_scale) {
   constexpr int L = D / 16;
+  const int which = (int)blockIdx.x >= sets.first;
+  const spx_head_norm& in = sets.set[which];
+  const uint16_t* __restrict__ const tok = reinterpret_cast<const uint16_t*>(in.tok);
+  const uint16_t* __restrict__ const gain = reinterpret_cast<const uint16_t*>(in.gain);
+  uint16_t* __restrict__ const out = reinterpret_cast<uint16_t*>(in.out);
+  uint16_t* __restrict__ const pass = reinterpret_cast<uint16_t*>(in.pass);
+  float* __restrict__ const rstd = in.rstd;
+  const int64_t* __restrict__ const pos = in.position_ids;
+  const int64_t ld = in.ld_tok, hs_out = in.out_head_stride, hs_pass = in.pass_head_stride;
+  const int T = (int)in.T, n_heads = in.n_heads, n_pass = in.n_pass;
+  const float eps = in.eps;
   const int heads = n_heads + n_pass, groups = (heads + HEADS - 1) / HEADS;
-  const int64_t item = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+  const int64_t item = (int64_t)((int)blockIdx.x - (which ? sets.first : 0)) * (256 / L) + threadIdx.x / L;
   if (item >= (int64_t)T * groups) return;  // (all lanes of a head together)
   const int hg = (int)(item % groups), t = (int)(item / groups);
   const int part = threadIdx.x % L, d0 = part * 8;
@@ -529,13 +540,22 @@ __global__ __launch_bounds__(256) void head_norm_rope_kernel(const uint16_t* __r
 // The way back: dtok from the head-major gradients (rotated back, then through the norm), and the gain's partial sums, one
 // row of D per workgroup (slots as spx_rmsnorm_bwd_slots; accumulate: they start from what dw_part holds).
 template <int D, int HEADS>
-__global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(
-    const uint16_t* __restrict__ tok, int64_t ld, const uint16_t* __restrict__ dout, int64_t hs_out,
-    const uint16_t* __restrict__ dpass, int64_t hs_pass, const int64_t* __restrict__ pos,
-    const float* __restrict__ inv_freq, const uint16_t* __restrict__ gain, const float* __restrict__ rstd,
-    uint16_t* __restrict__ dtok, int64_t ld_d, float* __restrict__ dw_part, int accumulate, int T, int n_heads, int n_pass,
-    int64_t pos_offset, float table_scale) {
+__global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(HeadSets sets, const float* __restrict__ inv_freq,
+                                                                 int64_t pos_offset, float table_scale) {
   constexpr int L = D / 16, PER = 256 / L;
+  const int which = (int)blockIdx.x >= sets.first;
+  const spx_head_norm& in = sets.set[which];
+  const uint16_t* __restrict__ const tok = reinterpret_cast<const uint16_t*>(in.tok);
+  const uint16_t* __restrict__ const gain = reinterpret_cast<const uint16_t*>(in.gain);
+  const uint16_t* __restrict__ const dout = reinterpret_cast<const uint16_t*>(in.out);
+  const uint16_t* __restrict__ const dpass = reinterpret_cast<const uint16_t*>(in.pass);
+  const float* __restrict__ const rstd = in.rstd;
+  const int64_t* __restrict__ const pos = in.position_ids;
+  uint16_t* __restrict__ const dtok = reinterpret_cast<uint16_t*>(in.dtok);
+  float* __restrict__ const dw_part = in.dw_scratch;
+  const int64_t ld = in.ld_tok, hs_out = in.out_head_stride, hs_pass = in.pass_head_stride, ld_d = in.ld_dtok;
+  const int T = (int)in.T, n_heads = in.n_heads, n_pass = in.n_pass, accumulate = in.accumulate;
+  const int block = (int)blockIdx.x - (which ? sets.first : 0), blocks = which ? (int)gridDim.x - sets.first : sets.first;
   __shared__ float red[PER * D];
   const int heads = n_heads + n_pass, groups = (heads + HEADS - 1) / HEADS;
   const int part = threadIdx.x % L, d0 = part * 8;
@@ -545,7 +565,7 @@ __global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(
   unpack8f(*reinterpret_cast<const u32x4*>(gain + D / 2 + d0), wb);
 #pragma unroll
   for (int e = 0; e < 8; ++e) dwa[e] = dwb[e] = 0.f;
-  for (int64_t item = (int64_t)blockIdx.x * PER + threadIdx.x / L; item < items; item += (int64_t)gridDim.x * PER) {
+  for (int64_t item = (int64_t)block * PER + threadIdx.x / L; item < items; item += (int64_t)blocks * PER) {
     const int hg = (int)(item % groups), t = (int)(item / groups);
     u32x4 ga[HEADS], gb[HEADS], xa[HEADS], xb[HEADS];
     float r[HEADS];
@@ -626,7 +646,7 @@ __global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(
   }
   __syncthreads();
   if (threadIdx.x < D) {
-    float* const o = dw_part + (int64_t)blockIdx.x * D + threadIdx.x;
+    float* const o = dw_part + (int64_t)block * D + threadIdx.x;
     float sum = accumulate ? *o : 0.f;
 #pragma unroll
     for (int k = 0; k < PER; ++k) sum += red[k * D + threadIdx.x];
@@ -1321,26 +1341,32 @@ static int head_norm_rope_checks(const char* fn, int64_t ld, int64_t T, int32_t 
 // heads per thread: as many as leave every compute unit two workgroups
 static int heads_per_thread(int64_t threads) { return threads >= 4 * 512 * 256 ? 4 : threads >= 2 * 512 * 256 ? 2 : 1; }
 
-extern "C" int spx_head_norm_rope(const void* tok, int64_t ld_tok, void* out, int64_t out_head_stride, void* pass,
-                                  int64_t pass_head_stride, const int64_t* position_ids, const float* inv_freq,
-                                  const void* gain, float* rstd, int64_t T, int32_t n_heads, int32_t n_pass, int32_t D,
-                                  int64_t position_offset, float table_scale, float eps, void* stream) {
-  const char* fn = __func__;
-  if (int rc = head_norm_rope_checks(fn, ld_tok, T, n_heads, n_pass, D, out_head_stride, pass_head_stride, table_scale))
-    return rc;
-  SPX_REQ_FN(tok && out && position_ids && inv_freq && gain && rstd && (!n_pass || pass), "null buffer");
-  SPX_REQ_FN(al16(tok) && al16(out) && al16(pass) && al16(gain), "buffers must be 16-byte aligned");
-  const int64_t threads = T * (n_heads + n_pass) * (D / 16);
-  const int per = heads_per_thread(threads);
-#define SPX_LAUNCH(DD, HEADS)                                                                                         \
-  hipLaunchKernelGGL((head_norm_rope_kernel<DD, HEADS>),                                                              \
-                     dim3((unsigned)((T * ((n_heads + n_pass + HEADS - 1) / HEADS) * (DD / 16) + 255) / 256)), dim3(256), \
-                     0, reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(tok), ld_tok,        \
-                     reinterpret_cast<uint16_t*>(out), out_head_stride, reinterpret_cast<uint16_t*>(pass),            \
-                     pass_head_stride, position_ids, inv_freq, reinterpret_cast<const uint16_t*>(gain), rstd, (int)T, \
-                     (int)n_heads, (int)n_pass, position_offset, table_scale, eps)
 #define SPX_LAUNCH_D(HEADS)                                                                                           \
   do { if (D == 64) SPX_LAUNCH(64, HEADS); else if (D == 128) SPX_LAUNCH(128, HEADS); else SPX_LAUNCH(256, HEADS); } while (0)
+
+static int head_norm_rope_launch(const char* fn, const spx_head_norm* sets, int32_t count, const float* inv_freq, int32_t D,
+                                 int64_t position_offset, float table_scale, void* stream) {
+  SPX_REQ_FN(sets && (count == 1 || count == 2) && inv_freq, "one or two sets of heads and their frequencies");
+  HeadSets hs{};
+  int64_t threads = 0;
+  for (int i = 0; i < count; ++i) {
+    const spx_head_norm& h = hs.set[i] = sets[i];
+    if (int rc = head_norm_rope_checks(fn, h.ld_tok, h.T, h.n_heads, h.n_pass, D, h.out_head_stride, h.pass_head_stride,
+                                       table_scale))
+      return rc;
+    SPX_REQ_FN(h.tok && h.out && h.position_ids && h.gain && h.rstd && (!h.n_pass || h.pass), "null buffer");
+    SPX_REQ_FN(al16(h.tok) && al16(h.out) && al16(h.pass) && al16(h.gain), "buffers must be 16-byte aligned");
+    threads += h.T * (h.n_heads + h.n_pass) * (D / 16);
+  }
+  const int per = heads_per_thread(threads);
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    blocks += (hs.set[i].T * ((hs.set[i].n_heads + hs.set[i].n_pass + per - 1) / per) * (D / 16) + 255) / 256;
+    if (i == 0) hs.first = (int)blocks;
+  }
+#define SPX_LAUNCH(DD, HEADS)                                                                                         \
+  hipLaunchKernelGGL((head_norm_rope_kernel<DD, HEADS>), dim3((unsigned)blocks), dim3(256), 0,                        \
+                     reinterpret_cast<hipStream_t>(stream), hs, inv_freq, position_offset, table_scale)
   if (per == 4) SPX_LAUNCH_D(4);
   else if (per == 2) SPX_LAUNCH_D(2);
   else SPX_LAUNCH_D(1);
@@ -1348,32 +1374,60 @@ extern "C" int spx_head_norm_rope(const void* tok, int64_t ld_tok, void* out, in
   return check_launch(fn);
 }
 
+static int head_norm_rope_bwd_launch(const char* fn, const spx_head_norm* sets, int32_t count, const float* inv_freq,
+                                     int32_t D, int64_t position_offset, float table_scale, void* stream) {
+  SPX_REQ_FN(sets && (count == 1 || count == 2) && inv_freq, "one or two sets of heads and their frequencies");
+  HeadSets hs{};
+  int64_t threads = 0, blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    const spx_head_norm& h = hs.set[i] = sets[i];
+    if (int rc = head_norm_rope_checks(fn, h.ld_tok, h.T, h.n_heads, h.n_pass, D, h.out_head_stride, h.pass_head_stride,
+                                       table_scale))
+      return rc;
+    SPX_REQ_FN(h.tok && h.out && h.position_ids && h.gain && h.rstd && h.dtok && (!h.n_pass || h.pass), "null buffer");
+    SPX_REQ_FN(al16(h.tok) && al16(h.out) && al16(h.pass) && al16(h.gain) && al16(h.dtok), "buffers must be 16-byte aligned");
+    SPX_REQ_FN(h.ld_dtok % 8 == 0 && h.ld_dtok >= (int64_t)(h.n_heads + h.n_pass) * D, "bad row stride of the gradient");
+    threads += h.T * (h.n_heads + h.n_pass) * (D / 16);
+    blocks += spx_rmsnorm_bwd_slots(h.T * h.n_heads, D);
+    if (i == 0) hs.first = (int)blocks;
+  }
+  const int per = heads_per_thread(threads);
+#define SPX_LAUNCH(DD, HEADS)                                                                                         \
+  hipLaunchKernelGGL((head_norm_rope_bwd_kernel<DD, HEADS>), dim3((unsigned)blocks), dim3(256), 0,                    \
+                     reinterpret_cast<hipStream_t>(stream), hs, inv_freq, position_offset, table_scale)
+  if (per >= 2) SPX_LAUNCH_D(2);
+  else SPX_LAUNCH_D(1);
+#undef SPX_LAUNCH
+#undef SPX_LAUNCH_D
+  return check_launch(fn);
+}
+
+extern "C" int spx_head_norm_rope_sets(const spx_head_norm* sets, int32_t count, const float* inv_freq, int32_t D,
+                                       int64_t position_offset, float table_scale, void* stream) {
+  return head_norm_rope_launch(__func__, sets, count, inv_freq, D, position_offset, table_scale, stream);
+}
+extern "C" int spx_head_norm_rope_bwd_sets(const spx_head_norm* sets, int32_t count, const float* inv_freq, int32_t D,
+                                           int64_t position_offset, float table_scale, void* stream) {
+  return head_norm_rope_bwd_launch(__func__, sets, count, inv_freq, D, position_offset, table_scale, stream);
+}
+extern "C" int spx_head_norm_rope(const void* tok, int64_t ld_tok, void* out, int64_t out_head_stride, void* pass,
+                                  int64_t pass_head_stride, const int64_t* position_ids, const float* inv_freq,
+                                  const void* gain, float* rstd, int64_t T, int32_t n_heads, int32_t n_pass, int32_t D,
+                                  int64_t position_offset, float table_scale, float eps, void* stream) {
+  const spx_head_norm set = {tok, ld_tok, out, out_head_stride, pass, pass_head_stride, position_ids, gain, rstd, T, n_heads,
+                             n_pass, eps, 0, nullptr, 0, nullptr};
+  return head_norm_rope_launch(__func__, &set, 1, inv_freq, D, position_offset, table_scale, stream);
+}
 extern "C" int spx_head_norm_rope_bwd(const void* tok, int64_t ld_tok, const void* dout, int64_t dout_head_stride,
                                       const void* dpass, int64_t dpass_head_stride, const int64_t* position_ids,
                                       const float* inv_freq, const void* gain, const float* rstd, void* dtok,
                                       int64_t ld_dtok, float* dw_scratch, int32_t accumulate, int64_t T, int32_t n_heads,
                                       int32_t n_pass, int32_t D, int64_t position_offset, float table_scale,
                                       void* stream) {
-  const char* fn = __func__;
-  if (int rc = head_norm_rope_checks(fn, ld_tok, T, n_heads, n_pass, D, dout_head_stride, dpass_head_stride, table_scale))
-    return rc;
-  SPX_REQ_FN(tok && dout && position_ids && inv_freq && gain && rstd && dtok && (!n_pass || dpass), "null buffer");
-  SPX_REQ_FN(al16(tok) && al16(dout) && al16(dpass) && al16(gain) && al16(dtok), "buffers must be 16-byte aligned");
-  SPX_REQ_FN(ld_dtok % 8 == 0 && ld_dtok >= (int64_t)(n_heads + n_pass) * D, "bad row stride of the gradient");
-  const int64_t slots = spx_rmsnorm_bwd_slots(T * n_heads, D);
-  const int per = heads_per_thread(T * (n_heads + n_pass) * (D / 16));
-#define SPX_LAUNCH(DD, HEADS)                                                                                         \
-  hipLaunchKernelGGL((head_norm_rope_bwd_kernel<DD, HEADS>), dim3((unsigned)slots), dim3(256), 0,                     \
-                     reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint16_t*>(tok), ld_tok,           \
-                     reinterpret_cast<const uint16_t*>(dout), dout_head_stride,                                       \
-                     reinterpret_cast<const uint16_t*>(dpass), dpass_head_stride, position_ids, inv_freq,             \
-                     reinterpret_cast<const uint16_t*>(gain), rstd, reinterpret_cast<uint16_t*>(dtok), ld_dtok,       \
-                     dw_scratch, (int)accumulate, (int)T, (int)n_heads, (int)n_pass, position_offset, table_scale)
-  if (per >= 2) SPX_LAUNCH_D(2);
-  else SPX_LAUNCH_D(1);
-#undef SPX_LAUNCH
-#undef SPX_LAUNCH_D
-  return check_launch(fn);
+  const spx_head_norm set = {tok, ld_tok, const_cast<void*>(dout), dout_head_stride, const_cast<void*>(dpass),
+                             dpass_head_stride, position_ids, gain, const_cast<float*>(rstd), T, n_heads, n_pass, 0.f,
+                             accumulate, dtok, ld_dtok, dw_scratch};
+  return head_norm_rope_bwd_launch(__func__, &set, 1, inv_freq, D, position_offset, table_scale, stream);
 }
 
 #undef SPX_REQ_FN

@@ -277,13 +277,12 @@ PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t 
                rk = at::empty({nk, hkv}, q_tok.options().dtype(at::kFloat));
   const Tensor k = kv.select(0, 0), v = kv.select(0, 1);
   const float* const f = inv_freq.const_data_ptr<float>();
-  check(spx_head_norm_rope(in(q_tok), q_tok.stride(0), to(q), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(), f,
-                           in(gain_q), floats(rq), nq, hq, 0, d, 0, table_scale, eps_q, st),
-        "spx_head_norm_rope");
-  check(spx_head_norm_rope(in(kv_tok) + kv_column, kv_tok.stride(0), to(k), nk * d, to(v), nk * d,
-                           kv_pos.const_data_ptr<int64_t>(), f, in(gain_k), floats(rk), nk, hkv, hkv, d, 0, table_scale,
-                           eps_k, st),
-        "spx_head_norm_rope");
+  const spx_head_norm sets[2] = {
+      {in(q_tok), q_tok.stride(0), to(q), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(), in(gain_q), floats(rq), nq,
+       (int32_t)hq, 0, (float)eps_q, 0, nullptr, 0, nullptr},
+      {in(kv_tok) + kv_column, kv_tok.stride(0), to(k), nk * d, to(v), nk * d, kv_pos.const_data_ptr<int64_t>(), in(gain_k),
+       floats(rk), nk, (int32_t)hkv, (int32_t)hkv, (float)eps_k, 0, nullptr, 0, nullptr}};
+  check(spx_head_norm_rope_sets(sets, 2, f, (int32_t)d, 0, (float)table_scale, st), "spx_head_norm_rope_sets");
   const Tensor att = rows_or_new(slot, nq, hq * d, q_tok);
   const Tensor lse = attention_forward(q, k, v, Mask{lo, hi, blo, bhi, T, step}, scaling, att);
   return tuple_of(released, {q, kv, rq, rk, att, lse});
@@ -312,14 +311,13 @@ PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t
   const Tensor dq_tok = rows_or_new(slot_q, nq, q_tok.size(1), q),
                dkv_tok = kv_column ? dq_tok : rows_or_new(slot_kv, nk, kv_tok.size(1), q);
   const float* const f = inv_freq.const_data_ptr<float>();
-  check(spx_head_norm_rope_bwd(in(q_tok), q_tok.stride(0), in(dq), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(),
-                               f, in(gain_q), floats(rq), to(dq_tok), dq_tok.stride(0), floats(scratch_q), acc_q, nq, hq,
-                               0, d, 0, table_scale, st),
-        "spx_head_norm_rope_bwd");
-  check(spx_head_norm_rope_bwd(in(kv_tok) + kv_column, kv_tok.stride(0), in(dk), nk * d, in(dv), nk * d,
-                               kv_pos.const_data_ptr<int64_t>(), f, in(gain_k), floats(rk), to(dkv_tok) + kv_column,
-                               dkv_tok.stride(0), floats(scratch_k), acc_k, nk, hkv, hkv, d, 0, table_scale, st),
-        "spx_head_norm_rope_bwd");
+  const spx_head_norm sets[2] = {
+      {in(q_tok), q_tok.stride(0), to(dq), nq * d, nullptr, 0, q_pos.const_data_ptr<int64_t>(), in(gain_q), floats(rq), nq,
+       (int32_t)hq, 0, 0.f, (int32_t)acc_q, to(dq_tok), dq_tok.stride(0), floats(scratch_q)},
+      {in(kv_tok) + kv_column, kv_tok.stride(0), to(dk), nk * d, to(dv), nk * d, kv_pos.const_data_ptr<int64_t>(), in(gain_k),
+       floats(rk), nk, (int32_t)hkv, (int32_t)hkv, 0.f, (int32_t)acc_k, to(dkv_tok) + kv_column, dkv_tok.stride(0),
+       floats(scratch_k)}};
+  check(spx_head_norm_rope_bwd_sets(sets, 2, f, (int32_t)d, 0, (float)table_scale, st), "spx_head_norm_rope_bwd_sets");
   return tuple_of(released, {dq_tok, dkv_tok});
   END_HANDLE_TH_ERRORS
 }
