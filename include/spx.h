@@ -588,6 +588,16 @@ int spx_rmsnorm_dweight(const float* dw_scratch, int64_t slots, int64_t H, void*
 int spx_rmsnorm_dweights(const float* const* dw_scratch, const int64_t* slots, const int64_t* H, void* const* dweight,
                          const int32_t* is_f32, int32_t count, void* stream);
 
+/* The same two with partial results in the place of b and of dy: parts tensors of rows x H fp32, one after the other, as
+ * spx_gemm_bf16_auto_parts leaves them; they are added in their order and rounded once to bf16, so the results are those of
+ * the product and the norm apart.  dw_scratch may be NULL (the gain does not train; dx is wanted then). */
+int spx_add_rmsnorm_fwd_parts(const void* a, int64_t ld_a, const float* partial, int32_t parts, void* sum,
+                              int64_t ld_sum, const void* weight, void* y, int64_t ld_y, float* rstd,
+                              int64_t rows, int64_t H, float eps, void* stream);
+int spx_rmsnorm_bwd_parts(const void* x, int64_t ld_x, const void* weight, const float* partial, int32_t parts,
+                          const void* dres, int64_t ld_dres, const float* rstd, void* dx, int64_t ld_dx,
+                          float* dw_scratch, int32_t accumulate, int64_t rows, int64_t H, void* stream);
+
 /* Two RMSNorms of one row count in one launch, written into the halves of y [rows, 2H] (row stride ld_y):
  * y[:, :H] = norm(a), y[:, H:] = norm(b); rstd [2, rows].  The backward of both (dy as y; dres_b, may be null,
  * is added to b's input gradient; da / db may be null: only the gain's gradient is wanted then) leaves the
@@ -741,6 +751,13 @@ int spx_gemm_auto_tile(int form, int64_t M, int64_t N, int64_t K, int32_t max_pa
 int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                        int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live,
                        int32_t max_parts, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The same without the pass that adds the parts where the whole contraction is cut: *parts (host memory, written before
+ * the return) is then their number and the workspace holds as many [M, N] fp32 tensors one after the other, c is not
+ * written; 1: c is.  Whatever is launched next on the stream reads them: the workspace serves the next product. */
+int spx_gemm_bf16_auto_parts(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                             int64_t ldc, int64_t M, int64_t N, int64_t K, int32_t max_parts, void* workspace,
+                             int64_t workspace_bytes, int32_t* parts, void* stream);
 
 /* spx_gemm_bf16_nt for products whose number of 256 x 256 output tiles leaves the last round of
  * workgroups mostly empty (384 tiles on 256 compute units: the second round is half empty and

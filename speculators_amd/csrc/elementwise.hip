@@ -46,6 +46,27 @@ __device__ __forceinline__ float block_sum(float v, float* lds) {
 // The kernel is bound by HBM where the rows fill the chip and by the launch below that: the two norms
 // of the first layer (PAIR) are one launch of twice the workgroups, the upper half of the grid's y
 // working on the second norm (T = 512, H = 2048: 3.7 us for the pair, 4.1 us for each one alone).
+// PARTS: that second tensor is a product whose contraction was cut (rows of H, one after the other; stride floats from
+// part to part): its partial results are added in their order and rounded here as the product's own last pass does, which
+// saves that launch and the rounded tensor's way out and back.  T = 512, H = 2048: forward, four parts, 4.7 us for the pass
+// and 4.3 for the norm before, 5.7 now; backward, eight parts, 6.6 and 5.5 before, 9.4 now (33 MB of partial results at
+// 3.6 TB/s; four parts' loads in flight by hand measured the same).
+struct NormParts {
+  const float* at;
+  int64_t stride;
+  int count;
+  __device__ __forceinline__ void sum(int64_t offset, float v[8]) const {
+    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+    const float* src = at + offset;
+    for (int p = 0; p < count; ++p, src += stride) {
+      lo += *reinterpret_cast<const f32x4*>(src);
+      hi += *reinterpret_cast<const f32x4*>(src + 4);
+    }
+    const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    unpack8f(pack8f(f), v);
+  }
+};
+
 struct NormFwdSet {
   const uint16_t* x;
   int64_t ld_x;
@@ -55,11 +76,11 @@ struct NormFwdSet {
   float* rstd;
 };
 
-template <int MAXC, bool WAVE_ROWS, bool RES = false, bool PAIR = false, int NT = 256>
+template <int MAXC, bool WAVE_ROWS, bool RES = false, bool PAIR = false, int NT = 256, bool PARTS = false>
 __global__ __launch_bounds__(NT) void rmsnorm_fwd_kernel(
     NormFwdSet one, NormFwdSet two, int64_t rows, int H,
     float eps, const uint16_t* __restrict__ res = nullptr, int64_t ld_res = 0,
-    uint16_t* __restrict__ sum = nullptr, int64_t ld_sum = 0) {
+    uint16_t* __restrict__ sum = nullptr, int64_t ld_sum = 0, NormParts parts = NormParts{}) {
   __shared__ float red[NT / 64];
   const bool second = PAIR && blockIdx.y;
   const uint16_t* __restrict__ x = second ? two.x : one.x;
@@ -81,7 +102,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_fwd_kernel(
       unpack8f(*reinterpret_cast<const u32x4*>(x + row * ld_x + ch * 8), v[c]);
       if (RES) {
         float b[8];
-        unpack8f(*reinterpret_cast<const u32x4*>(res + row * ld_res + ch * 8), b);
+        if (PARTS) parts.sum(row * H + ch * 8, b);
+        else unpack8f(*reinterpret_cast<const u32x4*>(res + row * ld_res + ch * 8), b);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[c][e] += b[e];
         const u32x4 packed = pack8f(v[c]);
@@ -135,8 +157,9 @@ struct NormBwdSet {
   int accumulate;
 };
 
-template <int MAXC, bool WAVE_ROWS, bool PAIR = false, int NT = 256>
-__global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(NormBwdSet one, NormBwdSet two, int64_t rows, int H) {
+template <int MAXC, bool WAVE_ROWS, bool PAIR = false, int NT = 256, bool PARTS = false>
+__global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(NormBwdSet one, NormBwdSet two, int64_t rows, int H,
+                                                         NormParts parts = NormParts{}) {
   __shared__ float red[WAVE_ROWS ? 4 * 512 : NT / 64];
   const bool second = PAIR && blockIdx.y;
   const uint16_t* __restrict__ x = second ? two.x : one.x;
@@ -179,7 +202,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(NormBwdSet one, NormBwd
       if (ch < nch) {
         float xv[8], dv[8];
         unpack8f(*reinterpret_cast<const u32x4*>(x + row * ld_x + ch * 8), xv);
-        unpack8f(*reinterpret_cast<const u32x4*>(dy + row * ld_dy + ch * 8), dv);
+        if (PARTS) parts.sum(row * H + ch * 8, dv);
+        else unpack8f(*reinterpret_cast<const u32x4*>(dy + row * ld_dy + ch * 8), dv);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           xh[c][e] = xv[e] * r;
@@ -952,7 +976,8 @@ extern "C" int64_t spx_rmsnorm_bwd_slots(int64_t rows, int64_t H) {
 
 static int rmsnorm_fwd_launch(const char* fn, const void* x, int64_t ld_x, const void* res, int64_t ld_res,
                               void* sum, int64_t ld_sum, const void* weight, void* y, int64_t ld_y,
-                              float* rstd, int64_t rows, int64_t H, float eps, void* stream) {
+                              float* rstd, int64_t rows, int64_t H, float eps, void* stream,
+                              const NormParts& parts = NormParts{}) {
   if (!(rows >= 0 && H > 0)) return fail_arg(fn, "bad sizes");
   if (!(H % 8 == 0 && ld_x % 8 == 0 && ld_y % 8 == 0 && ld_res % 8 == 0 && ld_sum % 8 == 0))
     return fail_arg(fn, "H and the row strides must be multiples of 8");
@@ -970,12 +995,15 @@ static int rmsnorm_fwd_launch(const char* fn, const void* x, int64_t ld_x, const
 #define SPX_LAUNCH(MAXC, WR, NT)                                                                             \
   do {                                                                                                       \
     const unsigned grid = (unsigned)(WR ? (rows + 3) / 4 : rows);                                            \
-    if (res)                                                                                                 \
+    if (parts.count)                                                                                         \
+      hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, true, false, NT, true>), dim3(grid), dim3(NT), 0, st, \
+                         set, set, rows, (int)H, eps, nullptr, 0, sp, ld_sum, parts);                        \
+    else if (res)                                                                                            \
       hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, true, false, NT>), dim3(grid), dim3(NT), 0, st, set,  \
-                         set, rows, (int)H, eps, rp, ld_res, sp, ld_sum);                                    \
+                         set, rows, (int)H, eps, rp, ld_res, sp, ld_sum, parts);                             \
     else                                                                                                     \
       hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, false, false, NT>), dim3(grid), dim3(NT), 0, st, set, \
-                         set, rows, (int)H, eps, nullptr, 0, nullptr, 0);                                    \
+                         set, rows, (int)H, eps, nullptr, 0, nullptr, 0, parts);                             \
   } while (0)
   SPX_NORM_FORMS(SPX_LAUNCH);
 #undef SPX_LAUNCH
@@ -996,6 +1024,22 @@ extern "C" int spx_add_rmsnorm_fwd(const void* a, int64_t ld_a, const void* b, i
                             stream);
 }
 
+// the rules of partial results in place of a bf16 tensor of rows of H
+static int parts_check(const char* fn, const float* partial, int32_t parts, int64_t rows, int64_t H) {
+  if (!(partial && al16(partial) && parts >= 1)) return fail_arg(fn, "null or unaligned partial results");
+  if (!(rows > 0 && H > 0 && H % 8 == 0)) return fail_arg(fn, "rows > 0 and H a multiple of 8");
+  return SPX_OK;
+}
+
+extern "C" int spx_add_rmsnorm_fwd_parts(const void* a, int64_t ld_a, const float* partial, int32_t parts, void* sum,
+                                         int64_t ld_sum, const void* weight, void* y, int64_t ld_y, float* rstd,
+                                         int64_t rows, int64_t H, float eps, void* stream) {
+  if (int rc = parts_check(__func__, partial, parts, rows, H)) return rc;
+  SPX_REQUIRE(sum, "null buffer");
+  return rmsnorm_fwd_launch(__func__, a, ld_a, nullptr, 0, sum, ld_sum, weight, y, ld_y, rstd, rows, H, eps, stream,
+                            NormParts{partial, rows * H, parts});
+}
+
 extern "C" int spx_rmsnorm_pair_fwd(const void* a, int64_t ld_a, const void* weight_a, const void* b, int64_t ld_b,
                                     const void* weight_b, void* y, int64_t ld_y, float* rstd, int64_t rows,
                                     int64_t H, float eps, void* stream) {
@@ -1013,7 +1057,7 @@ extern "C" int spx_rmsnorm_pair_fwd(const void* a, int64_t ld_a, const void* wei
                           yp + H, ld_y, rstd + rows};
 #define SPX_LAUNCH(MAXC, WR, NT)                                                                                 \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<MAXC, WR, false, true, NT>), dim3((unsigned)(WR ? (rows + 3) / 4 : rows), 2), \
-                     dim3(NT), 0, st, one, two, rows, (int)H, eps, nullptr, 0, nullptr, 0)
+                     dim3(NT), 0, st, one, two, rows, (int)H, eps, nullptr, 0, nullptr, 0, NormParts{})
   SPX_NORM_FORMS(SPX_LAUNCH);
 #undef SPX_LAUNCH
   return check_launch(__func__);
@@ -1022,12 +1066,13 @@ extern "C" int spx_rmsnorm_pair_fwd(const void* a, int64_t ld_a, const void* wei
 static int rmsnorm_bwd_launch(const char* fn, const void* x, int64_t ld_x, const void* weight, const void* dy,
                               int64_t ld_dy, const void* dres, int64_t ld_dres, const float* rstd, void* dx,
                               int64_t ld_dx, void* dweight, float* dw_scratch, int64_t rows, int64_t H,
-                              void* stream, bool partial_only = false, int accumulate = 0) {
+                              void* stream, bool partial_only = false, int accumulate = 0,
+                              const NormParts& parts = NormParts{}) {
   if (!(rows > 0 && H > 0)) return fail_arg(fn, "bad sizes");
   if (!(H % 8 == 0 && ld_x % 8 == 0 && ld_dy % 8 == 0 && ld_dx % 8 == 0 && ld_dres % 8 == 0))
     return fail_arg(fn, "H and the row strides must be multiples of 8");
   if (H > 16384) return fail_arg(fn, "H must be at most 16384");
-  if (!(x && weight && dy && rstd)) return fail_arg(fn, "null buffer");
+  if (!(x && weight && (dy || parts.count) && rstd)) return fail_arg(fn, "null buffer");
   if (!(dx || dweight || partial_only)) return fail_arg(fn, "neither dx nor dweight requested");
   if (partial_only && !dw_scratch) return fail_arg(fn, "null dw_scratch");
   if (dres && !dx) return fail_arg(fn, "a residual gradient needs dx");
@@ -1041,9 +1086,15 @@ static int rmsnorm_bwd_launch(const char* fn, const void* x, int64_t ld_x, const
                           reinterpret_cast<const uint16_t*>(dy), ld_dy, rstd, reinterpret_cast<uint16_t*>(dx), ld_dx,
                           part, reinterpret_cast<const uint16_t*>(dres), ld_dres, accumulate};
   const int64_t slots = spx_rmsnorm_bwd_slots(rows, H);
-#define SPX_LAUNCH(MAXC, WR, NT)                                                                                    \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, false, NT>), dim3((unsigned)slots), dim3(NT), 0, st, set, set, \
-                     rows, (int)H)
+#define SPX_LAUNCH(MAXC, WR, NT)                                                                                         \
+  do {                                                                                                                   \
+    if (parts.count)                                                                                                     \
+      hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, false, NT, true>), dim3((unsigned)slots), dim3(NT), 0, st, set,   \
+                         set, rows, (int)H, parts);                                                                      \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, false, NT>), dim3((unsigned)slots), dim3(NT), 0, st, set, set,    \
+                         rows, (int)H, parts);                                                                           \
+  } while (0)
   SPX_NORM_FORMS(SPX_LAUNCH);
 #undef SPX_LAUNCH
   if (dweight)
@@ -1075,7 +1126,7 @@ extern "C" int spx_rmsnorm_pair_bwd_partial(const void* a, int64_t ld_a, const v
   const int64_t slots = spx_rmsnorm_bwd_slots(rows, H);
 #define SPX_LAUNCH(MAXC, WR, NT)                                                                                      \
   hipLaunchKernelGGL((rmsnorm_bwd_kernel<MAXC, WR, true, NT>), dim3((unsigned)slots, 2), dim3(NT), 0, st, one, two, \
-                     rows, (int)H)
+                     rows, (int)H, NormParts{})
   SPX_NORM_FORMS(SPX_LAUNCH);
 #undef SPX_LAUNCH
   return check_launch(__func__);
@@ -1102,6 +1153,14 @@ extern "C" int spx_rmsnorm_bwd_partial(const void* x, int64_t ld_x, const void* 
                                        int64_t rows, int64_t H, void* stream) {
   return rmsnorm_bwd_launch(__func__, x, ld_x, weight, dy, ld_dy, dres, ld_dres, rstd, dx, ld_dx, nullptr,
                             dw_scratch, rows, H, stream, true, accumulate != 0);
+}
+
+extern "C" int spx_rmsnorm_bwd_parts(const void* x, int64_t ld_x, const void* weight, const float* partial, int32_t parts,
+                                     const void* dres, int64_t ld_dres, const float* rstd, void* dx, int64_t ld_dx,
+                                     float* dw_scratch, int32_t accumulate, int64_t rows, int64_t H, void* stream) {
+  if (int rc = parts_check(__func__, partial, parts, rows, H)) return rc;
+  return rmsnorm_bwd_launch(__func__, x, ld_x, weight, nullptr, 0, dres, ld_dres, rstd, dx, ld_dx, nullptr, dw_scratch, rows,
+                            H, stream, dw_scratch != nullptr, accumulate != 0, NormParts{partial, rows * H, parts});
 }
 
 extern "C" int spx_rmsnorm_dweight(const float* dw_scratch, int64_t slots, int64_t H, void* dweight,

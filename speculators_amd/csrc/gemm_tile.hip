@@ -505,10 +505,11 @@ extern "C" int spx_gemm_auto_tile(int form, int64_t M, int64_t N, int64_t K, int
   return tile::choose(form, M, N, K, max_parts, can_split(N)).tile;
 }
 
-extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
-                                  int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live,
-                                  int32_t max_parts, void* workspace, int64_t workspace_bytes, void* stream) {
-  const char* fname = __func__;
+// left: where the number of partial results goes that are left in the workspace (NULL: they are added here)
+static int auto_product(const char* fname, int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                        int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live, int32_t max_parts,
+                        void* workspace, int64_t workspace_bytes, int32_t* left, void* stream) {
+  if (left) *left = 1;
   SPX_REQ_FN(max_parts >= 1 && max_parts <= 8, "max_parts must be 1 .. 8");
   if (int rc = tile::dense_check(fname, form, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
   const bool vec = ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;  // (what the pass that adds the parts stores)
@@ -538,7 +539,27 @@ extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const vo
   if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st))
     return rc;
   if (ch.parts == 1) return SPX_OK;
+  if (left) {
+    *left = ch.parts;
+    return SPX_OK;
+  }
   return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st);
+}
+
+extern "C" int spx_gemm_bf16_auto(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                                  int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live,
+                                  int32_t max_parts, void* workspace, int64_t workspace_bytes, void* stream) {
+  return auto_product(__func__, form, a, lda, b, ldb, c, ldc, M, N, K, m_live, max_parts, workspace, workspace_bytes, nullptr,
+                      stream);
+}
+
+extern "C" int spx_gemm_bf16_auto_parts(int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                                        int64_t ldc, int64_t M, int64_t N, int64_t K, int32_t max_parts, void* workspace,
+                                        int64_t workspace_bytes, int32_t* parts, void* stream) {
+  const char* fname = __func__;
+  SPX_REQ_FN(parts, "null buffer");
+  return auto_product(fname, form, a, lda, b, ldb, c, ldc, M, N, K, nullptr, max_parts, workspace, workspace_bytes, parts,
+                      stream);
 }
 
 // The weights in the product's own epilogue (a load per row and a multiply per result) or in the pass that adds its parts; the

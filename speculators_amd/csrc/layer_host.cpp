@@ -66,6 +66,26 @@ Tensor grad_rows(const Tensor& g) {
   return x.stride(1) == 1 ? x : x.contiguous();
 }
 
+// A product's result: stored, or (count > 1) as that many partial results in the thread's workspace, which the next launch
+// reads.
+struct Parted {
+  Tensor stored;
+  const float* at = nullptr;
+  int32_t count = 1;
+};
+
+// sum = a + b, y = its norm
+void add_norm(const Tensor& a, const Parted& b, const Tensor& sum, const Tensor& gain, const Tensor& y, float* rstd, double eps,
+              void* st) {
+  const int64_t rows = a.size(0), h = a.size(1);
+  if (b.count > 1)
+    check(spx_add_rmsnorm_fwd_parts(in(a), a.stride(0), b.at, b.count, to(sum), h, in(gain), to(y), h, rstd, rows, h, eps, st),
+          "spx_add_rmsnorm_fwd_parts");
+  else
+    check(spx_add_rmsnorm_fwd(in(a), a.stride(0), in(b.stored), h, to(sum), h, in(gain), to(y), h, rstd, rows, h, eps, st),
+          "spx_add_rmsnorm_fwd");
+}
+
 // The backward of a norm over x [rows, h], dres (may be undefined) added to dx; the partial sums of the gain's gradient go
 // to scratch (undefined: the gain does not train).
 void norm_backward(const Tensor& x, const Tensor& gain, const Tensor& dy, const Tensor& dres, const float* rstd,
@@ -80,6 +100,15 @@ void norm_backward(const Tensor& x, const Tensor& gain, const Tensor& dy, const 
     check(spx_add_rmsnorm_bwd(in(x), h, in(gain), in(dy), dy.stride(0), res, ld_dres, rstd, to(dx), h, nullptr, nullptr, rows,
                               h, st),
           "spx_add_rmsnorm_bwd");
+}
+
+void norm_backward(const Tensor& x, const Tensor& gain, const Parted& dy, const Tensor& dres, const float* rstd,
+                   const Tensor& dx, const Tensor& scratch, int64_t accumulate, void* st) {
+  if (dy.count == 1) return norm_backward(x, gain, dy.stored, dres, rstd, dx, scratch, accumulate, st);
+  const int64_t rows = x.size(0), h = x.size(1);
+  check(spx_rmsnorm_bwd_parts(in(x), h, in(gain), dy.at, dy.count, dres.defined() ? in(dres) : nullptr,
+                              dres.defined() ? dres.stride(0) : 0, rstd, to(dx), h, floats(scratch), accumulate, rows, h, st),
+        "spx_rmsnorm_bwd_parts");
 }
 
 // How gemm.py routed a product (``Route`` there)
@@ -105,6 +134,17 @@ struct Products {
       check(spx_gemm_bf16_auto(route, in(a), a.stride(0), in(b), b.stride(0), to(out), n, m, n, k,
                                m_live.defined() ? m_live.const_data_ptr<int32_t>() : nullptr, parts, w, wb, st),
             "spx_gemm_bf16_auto");
+    return out;
+  }
+  // for a launch that adds the parts of a cut product itself
+  Parted parted(int64_t route, const Tensor& a, const Tensor& b) const {
+    if ((route != kAutoNT && route != kAutoNN) || !ws.defined()) return {(*this)(route, a, b)};
+    const int64_t m = a.size(0), k = a.size(1), n = route == kAutoNN ? b.size(1) : b.size(0);
+    TORCH_CHECK_VALUE(b.size(route == kAutoNN ? 0 : 1) == k, "shape mismatch: a ", a.sizes(), " b ", b.sizes());
+    Parted out{at::empty({m, n}, a.options()), ws.const_data_ptr<float>()};
+    check(spx_gemm_bf16_auto_parts(route, in(a), a.stride(0), in(b), b.stride(0), to(out.stored), n, m, n, k, parts,
+                                   ws.mutable_data_ptr(), ws.nbytes(), &out.count, stream_of(a)),
+          "spx_gemm_bf16_auto_parts");
     return out;
   }
 };
@@ -139,17 +179,14 @@ PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n)
   void* const st = stream_of(residual);
   const Tensor stats = at::empty({2, t}, residual.options().dtype(at::kFloat));
   float* const rstd = floats(stats);
-  const Tensor o = product(r_o, att, wo);
+  const Parted o = product.parted(r_o, att, wo);
   const Tensor mid = at::empty({t, h}, residual.options()), z = rows_or_new(slot_gu, t, h, residual);
-  check(spx_add_rmsnorm_fwd(in(residual), residual.stride(0), in(o), h, to(mid), h, in(gain_post), to(z), h, rstd, t, h,
-                            eps_post, st),
-        "spx_add_rmsnorm_fwd");
+  add_norm(residual, o, mid, gain_post, z, rstd, eps_post, st);
   const Tensor gu = product(r_gu, z, wgu), act = rows_or_new(slot_d, t, f, residual);
   check(spx_swiglu_rows_fwd(in(gu), 2 * f, in(gu) + f, 2 * f, to(act), f, t, f, st), "spx_swiglu_rows_fwd");
-  const Tensor m = product(r_d, act, wd);
+  const Parted m = product.parted(r_d, act, wd);
   const Tensor y = at::empty({t, h}, residual.options()), normed = rows_or_new(slot_next, t, h, residual);
-  check(spx_add_rmsnorm_fwd(in(mid), h, in(m), h, to(y), h, in(gain_next), to(normed), h, rstd + t, t, h, eps_next, st),
-        "spx_add_rmsnorm_fwd");
+  add_norm(mid, m, y, gain_next, normed, rstd + t, eps_next, st);
   return tuple_of(released, {mid, stats, z, gu, act, y, normed});
   END_HANDLE_TH_ERRORS
 }
@@ -182,7 +219,8 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   const Tensor dact = product(r_d, dm, bd), dgu = rows_or_new(slot_gu, t, 2 * f, y);
   check(spx_swiglu_rows_bwd(in(gu), 2 * f, in(gu) + f, 2 * f, in(dact), f, to(dgu), 2 * f, to(dgu) + f, 2 * f, t, f, st),
         "spx_swiglu_rows_bwd");
-  const Tensor dz = product(r_gu, dgu, bgu), da = rows_or_new(slot_o, t, h, y);
+  const Parted dz = product.parted(r_gu, dgu, bgu);
+  const Tensor da = rows_or_new(slot_o, t, h, y);
   norm_backward(mid, gain_post, dz, dm, rstd, da, scratch_post, acc_post, st);
   return tuple_of(released, {dm, dgu, da, product(r_o, da, bo)});
   END_HANDLE_TH_ERRORS
