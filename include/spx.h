@@ -620,7 +620,7 @@ int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_stride, void
                  int32_t hq, int32_t hkv, int32_t D, int32_t rotary_dim, int32_t inverse,
                  int64_t position_offset, float table_scale, void* stream);
 
-/* count (1 .. 4) matrices of elements[i] values (multiples of 8), bf16 or (is_f32[i]) fp32, one after the other into out
+/* count (1 .. 8) matrices of elements[i] values (multiples of 8), bf16 or (is_f32[i]) fp32, one after the other into out
  * as bf16 (round to nearest even).  The three arrays are host memory, read before the call returns. */
 int spx_cat_bf16(const void* const* srcs, const int64_t* elements, const int32_t* is_f32, int32_t count, void* out,
                  void* stream);

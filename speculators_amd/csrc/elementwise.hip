@@ -679,22 +679,72 @@ __global__ __launch_bounds__(256) void head_norm_rope_bwd_kernel(HeadSets sets, 
 }
 
 // ---------------------------------------------------------------- weight staging
-// Up to four matrices of one width, bf16 or fp32, one after the other as bf16: the merged compute weights of a forward (q, k
-// and v; gate and up), and the bf16 copy of an fp32 master weight.  Bound by HBM; a thread has kCastAhead chunks of eight on
+// Up to eight matrices, bf16 or fp32, one after the other as bf16: the merged compute weights of a forward (q, k
+// and v; gate and up), and the bf16 copies of fp32 master weights, all of a layer's in one launch.  Bound by HBM; a thread has kCastAhead chunks of eight on
 // their way before it stores the first.  ONCE: more than the 256 MB of the last-level cache is read and written, loads that
 // nothing reads again leave it alone (gate and up of the 8B shape from fp32, 705 MB: 112 us, 128 without; two 8192 x 2048
-// matrices, 201 MB: 37 us, 30 without).  q, k and v of the 1B shape from fp32: 21 us in three copies -> 12.
-constexpr int kCastAhead = 4;
+// matrices, 201 MB: 37 us, 30 without).  q, k and v of the 1B shape from fp32: 21 us in three copies -> 12.  A workgroup
+// whose chunks are of one part takes it in scalar registers and loads without conditions (two 8192 x 2048 from fp32 36.2 ->
+// 31.6 us, 8192 x 8192 and two of 1024 rows 52.7 -> 49.8, 2048 x 2048 5.8 -> 5.2; bf16 sources the same); parts chosen by
+// an index into the arguments: three times the time.
+constexpr int kCastAhead = 4, kCastParts = 8;
 struct CastArgs {
-  const void* src[4];
-  int64_t end[4];  // chunks of eight, running
-  int f32;         // bit i: src[i] is fp32
+  const void* src[kCastParts];
+  int64_t end[kCastParts];  // chunks of eight, running
+  int f32;                  // bit i: src[i] is fp32
 };
 template <bool ONCE>
 __global__ __launch_bounds__(256) void cat_bf16_kernel(CastArgs p, u32x4* __restrict__ out, int64_t n) {
-  const int64_t i0 = ((int64_t)blockIdx.x * kCastAhead) * 256 + threadIdx.x;
+  const int64_t first = (int64_t)blockIdx.x * kCastAhead * 256, last = min(first + kCastAhead * 256, n) - 1;
+  const int64_t i0 = first + threadIdx.x;
   auto load = [](const u32x4* q) { return ONCE ? __builtin_nontemporal_load(q) : *q; };
+  auto cast = [](u32x4 a, u32x4 b) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = __uint_as_float(a[e]);
+      v[4 + e] = __uint_as_float(b[e]);
+    }
+    return pack8f(v);
+  };
+  auto part_of = [&](int64_t i) {
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < kCastParts - 1; ++k) s += i >= p.end[k];
+    return s;
+  };
+  // (constant indices only: the arguments stay in scalar registers)
+  auto pick = [&](int s, int64_t i) {
+    const void* src = p.src[0];
+    int64_t begin = 0;
+#pragma unroll
+    for (int k = 1; k < kCastParts; ++k) {
+      src = s == k ? p.src[k] : src;
+      begin = s == k ? p.end[k - 1] : begin;
+    }
+    return reinterpret_cast<const u32x4*>(src) + ((p.f32 >> s) & 1 ? 2 : 1) * (i - begin);
+  };
   u32x4 lo[kCastAhead], hi[kCastAhead];
+  const int s0 = part_of(first);
+  if (first + kCastAhead * 256 <= n && part_of(last) == s0) {  // whole workgroups of one part: nearly all
+    if ((p.f32 >> s0) & 1) {
+      const u32x4* const src = pick(s0, first) + 2 * threadIdx.x;
+#pragma unroll
+      for (int u = 0; u < kCastAhead; ++u) {
+        lo[u] = load(src + u * 512);
+        hi[u] = load(src + u * 512 + 1);
+      }
+#pragma unroll
+      for (int u = 0; u < kCastAhead; ++u) out[i0 + u * 256] = cast(lo[u], hi[u]);
+    } else {
+      const u32x4* const src = pick(s0, first) + threadIdx.x;
+#pragma unroll
+      for (int u = 0; u < kCastAhead; ++u) lo[u] = load(src + u * 256);
+#pragma unroll
+      for (int u = 0; u < kCastAhead; ++u) out[i0 + u * 256] = lo[u];
+    }
+    return;
+  }
   bool wide[kCastAhead];
 #pragma unroll
   for (int u = 0; u < kCastAhead; ++u) {
@@ -702,34 +752,17 @@ __global__ __launch_bounds__(256) void cat_bf16_kernel(CastArgs p, u32x4* __rest
     lo[u] = hi[u] = u32x4{0, 0, 0, 0};
     wide[u] = false;
     if (i < n) {
-      const int s = (i >= p.end[0]) + (i >= p.end[1]) + (i >= p.end[2]);
-      const void* const src = s == 0 ? p.src[0] : s == 1 ? p.src[1] : s == 2 ? p.src[2] : p.src[3];
-      const int64_t c = i - (s == 0 ? 0 : s == 1 ? p.end[0] : s == 2 ? p.end[1] : p.end[2]);
+      const int s = part_of(i);
+      const u32x4* const src = pick(s, i);
       wide[u] = (p.f32 >> s) & 1;
-      if (wide[u]) {
-        const u32x4* const f = reinterpret_cast<const u32x4*>(src) + 2 * c;
-        lo[u] = load(f);
-        hi[u] = load(f + 1);
-      } else {
-        lo[u] = load(reinterpret_cast<const u32x4*>(src) + c);
-      }
+      lo[u] = load(src);
+      if (wide[u]) hi[u] = load(src + 1);
     }
   }
 #pragma unroll
   for (int u = 0; u < kCastAhead; ++u) {
     const int64_t i = i0 + u * 256;
-    if (i >= n) continue;
-    if (wide[u]) {
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = __uint_as_float(lo[u][e]);
-        v[4 + e] = __uint_as_float(hi[u][e]);
-      }
-      out[i] = pack8f(v);
-    } else {
-      out[i] = lo[u];
-    }
+    if (i < n) out[i] = wide[u] ? cast(lo[u], hi[u]) : lo[u];
   }
 }
 
@@ -1357,11 +1390,11 @@ extern "C" int spx_rope_qkv(void* tok, int64_t ld_tok, void* q, int64_t q_head_s
 extern "C" int spx_cat_bf16(const void* const* srcs, const int64_t* elements, const int32_t* is_f32, int32_t count,
                             void* out, void* stream) {
   const char* fn = __func__;
-  SPX_REQ_FN(srcs && elements && is_f32 && count >= 1 && count <= 4, "one to four matrices");
+  SPX_REQ_FN(srcs && elements && is_f32 && count >= 1 && count <= kCastParts, "one to eight matrices");
   SPX_REQ_FN(out && al16(out), "null or unaligned buffer");
   CastArgs p{};
   int64_t n = 0;
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < kCastParts; ++i) {
     if (i < count) {
       SPX_REQ_FN(srcs[i] && al16(srcs[i]) && elements[i] > 0 && elements[i] % 8 == 0,
                  "null or unaligned matrix, or a size that is not a multiple of 8");

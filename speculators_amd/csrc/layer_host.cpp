@@ -624,11 +624,11 @@ PyObject* spx_layer_loss_steps_end(PyObject*, PyObject* const* args, Py_ssize_t 
 // The row-wise concatenation of one to four matrices as one bf16 matrix
 PyObject* spx_layer_cat_bf16(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK_TYPE(n >= 1 && n <= 4, "cat_bf16 takes one to four tensors");
+  TORCH_CHECK_TYPE(n >= 1 && n <= 8, "cat_bf16 takes one to eight tensors");
   Args x("cat_bf16", args, n, n);
-  const void* src[4];
-  int64_t elements[4], rows = 0;
-  int32_t f32[4];
+  const void* src[8];
+  int64_t elements[8], rows = 0;
+  int32_t f32[8];
   Tensor first;
   for (Py_ssize_t i = 0; i < n; ++i) {
     const Tensor& t = x.tensor();

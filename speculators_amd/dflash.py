@@ -169,9 +169,9 @@ class DFlashDecoderLayer(nn.Module):
         if (next_norm is None or not LY.untouched(att, self.mlp) or not LY.untouched(att.q_norm, att.k_norm)
                 or not LY.NormedLayer.takes(att, inv_freq, A.dflash_hip_attention_forward)):
             return None
-        W = self._stager.get
-        ws = (W(att.q_proj.weight), W(att.k_proj.weight, att.v_proj.weight), W(att.o_proj.weight),
-              W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight), W(self.mlp.down_proj.weight))
+        mlp = self.mlp
+        ws = self._stager.get_all((att.q_proj.weight,), (att.k_proj.weight, att.v_proj.weight), (att.o_proj.weight,),
+                                  (mlp.gate_proj.weight, mlp.up_proj.weight), (mlp.down_proj.weight,))
         if torch.is_grad_enabled() and not all(w.trainable for w in ws):
             return None
         return LY.NormedLayer(*ws, (0.0, att.q_norm.eps, att.k_norm.eps, self.post_attention_layernorm.eps,

@@ -190,9 +190,9 @@ class DecoderLayer(nn.Module):
                 or att.attn_fn is not A.ttt_hip_attention_forward or att.d not in A.KERNEL_HEAD_DIMS
                 or not cache.get("steps") or (self.first and cfg.norm_before_residual)):
             return None
-        W = self._stager.get
-        ws = (self._wqkv(), W(att.o_proj.weight), W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight),
-              W(self.mlp.down_proj.weight))
+        mlp = self.mlp
+        ws = self._stager.get_all((att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), (att.o_proj.weight,),
+                                  (mlp.gate_proj.weight, mlp.up_proj.weight), (mlp.down_proj.weight,))
         if torch.is_grad_enabled() and not all(w.trainable for w in ws):
             return None
         kvc = cache.get("kv")

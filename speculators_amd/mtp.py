@@ -154,9 +154,9 @@ class MTPLayer(nn.Module):
                 or not LY.untouched(att.q_norm, att.k_norm)
                 or not LY.NormedLayer.takes(att, inv_freq, A.ttt_hip_attention_forward)):
             return None
-        W = self._stager.get
-        ws = (W(att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), None, W(att.o_proj.weight),
-              W(self.mlp.gate_proj.weight, self.mlp.up_proj.weight), W(self.mlp.down_proj.weight))
+        mlp = self.mlp
+        ws = self._stager.get_all((att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), None, (att.o_proj.weight,),
+                                  (mlp.gate_proj.weight, mlp.up_proj.weight), (mlp.down_proj.weight,))
         if torch.is_grad_enabled() and not all(w is None or w.trainable for w in ws):
             return None
         eps = (self.input_layernorm.eps, att.q_norm.eps, att.k_norm.eps, self.post_attention_layernorm.eps,
