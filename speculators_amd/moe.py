@@ -266,10 +266,11 @@ class _Picked:
 
     @staticmethod
     def takes(x2, rows: int, experts: int) -> bool:
-        """Whether ``x2``'s rows are picked (else they are copied into sorted order first): few rows an expert (above 256
-        the products take tall tiles, are bound by their arithmetic and have no picked form) and a matrix that 32-bit
-        offsets reach."""
-        return 0 < rows <= PICK_ROWS * experts and x2.shape[0] * x2.shape[1] * 2 < PICK_BYTES
+        """Whether ``x2``'s rows are picked (else they are copied into sorted order first, by a launch with rules of its own
+        for strides and alignment): few rows an expert (above 256 the products take tall tiles, are bound by their
+        arithmetic and have no picked form) and a matrix that 32-bit offsets reach once it is contiguous."""
+        return (0 < rows <= PICK_ROWS * experts and x2.shape[0] * x2.shape[1] * 2 < PICK_BYTES
+                and x2.stride(0) >= x2.shape[1] and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0)
 
     def rows_of(self, form: int, a, b, picked: bool):
         """``a[src_row]`` (``picked``) or ``a`` times every expert's ``b.T`` (form 0) or ``b`` (form 1)."""
@@ -323,11 +324,12 @@ class _ExpertsMLP(torch.autograd.Function):
         stack_gu, use_gu = _ExpertStacks.use(st_gu, rows, h, i2)
         stack_dn, use_dn = _ExpertStacks.use(st_dn, rows, inter, h)
         picked = None
+        if x2.stride(1) != 1:
+            x2 = x2.contiguous()
         if stack_gu is None and stack_dn is None and _Picked.takes(x2, rows, e):
-            if x2.stride(1) != 1:
-                x2 = x2.contiguous()
-            picked, xs = _Picked(src_row, off), x2
-            hid = picked.rows_of(0, x2, w_gu, True)
+            # (the products' 32-bit offsets span the rows as they lie: of a column slice of a wide buffer, a copy is picked)
+            picked, xs = _Picked(src_row, off), x2.contiguous()
+            hid = picked.rows_of(0, xs, w_gu, True)
         else:
             xs = gather_rows(x2, src_row, out=None if stack_gu is None else stack_gu.x_slot(use_gu))
             hid = gemm_nt_grouped(xs, w_gu, off)
