@@ -1,4 +1,4 @@
-"""Tokens that the experts take: column slices of a wide buffer."""
+"""Tokens that the experts take: column slices of a wide buffer, and tokens that the caller writes to afterwards."""
 
 import pytest
 import torch
@@ -40,4 +40,22 @@ def test_column_slice(width, grad):
         for x2 in (x, wide[:, :H]):
             y = moe.experts_mlp(x2, scores, idx, *_staged(gate_up, down))
             got.append([y, *(torch.autograd.grad(y, (gate_up, down), torch.ones_like(y)) if grad else ())])
+    assert all(torch.equal(a, b) for a, b in zip(*got, strict=True))
+
+
+@pytest.mark.parametrize("trains", [True, False])
+def test_tokens_written_to_before_the_backward(trains):
+    from speculators_amd import moe
+
+    gate_up, down, x, scores, idx = _parts(70)
+    gate_up.requires_grad_(trains)
+    x.requires_grad_(True)
+    leaves = (x, gate_up, down) if trains else (x, down)
+    got = []
+    for write in (False, True):
+        x2 = x * 1.0
+        y = moe.experts_mlp(x2, scores, idx, *_staged(gate_up, down))
+        if write:
+            x2.zero_()
+        got.append(torch.autograd.grad(y, leaves, torch.ones_like(y)))
     assert all(torch.equal(a, b) for a, b in zip(*got, strict=True))
