@@ -785,13 +785,14 @@ class _HeadLabelCE(torch.autograd.Function):
     no gradient of their own."""
 
     @staticmethod
-    def forward(ctx, x2, weight, weight_t, labels, ignore_index, epilogue_stats=False, one_pass=False):
+    def forward(ctx, x2, weight, weight_t, labels, ignore_index, epilogue_stats=False, room=None):
         from .gemm import gemm_nt_stats, matmul_nt
 
         ctx.one_pass = False
-        if one_pass and not epilogue_stats:
+        one_pass = room is not None and not epilogue_stats  # room: GradientRoom, where the one-read pass takes the rows
+        if one_pass:
             logits = matmul_nt(x2, weight)
-            packed = _room_for_gradient(logits)
+            packed = room.take(logits)
             if packed is not None:
                 ctx.one_pass = True
                 rows, vocab = logits.shape
@@ -856,7 +857,7 @@ class _HeadLabelCE(torch.autograd.Function):
         return (_unpack_rows(dx_packed, row_map, rows),) + (None,) * 6
 
 
-def _label_one_pass(x2, weight, weight_t) -> bool:
+def _label_one_pass(x2, weight) -> bool:
     """Whether the row pass of the frozen-head cross-entropy leaves the logits gradient behind
     (``spx_label_ce_fwd_grad``): rows that fit a workgroup's registers and give every thread eight chunks at least."""
     vocab = weight.shape[0]
@@ -864,19 +865,40 @@ def _label_one_pass(x2, weight, weight_t) -> bool:
             and 0 < x2.shape[0] < 1 << 31)
 
 
-# of the card's memory, what one call's gradient may take from its forward to its backward
-LABEL_GRADIENT_SHARE = 1 / 24
+# of the memory that is available at a call, what the logits gradients of this call and of those still to come in the same
+# forward may take from their forward to their backward.  The logits of the calls to come take as much again, and half is
+# left for what the two-pass form needs as well: the activations of the layers in between (of a row, 60 KB beside 300 KB of
+# logits at 2048 -> 151936 and 250 KB beside 130 KB at 5120 -> 65536, the widest for its logits), and the backward
+LABEL_GRADIENT_SHARE = 1 / 4
 
 
-def _room_for_gradient(logits):
-    """Where the logits gradient waits for the backward, or None: it is made there then, from the logits."""
-    total = torch.cuda.get_device_properties(logits.device).total_memory
-    if logits.numel() * 2 > total * LABEL_GRADIENT_SHARE:
-        return None
+def _available_memory(device) -> int:
+    """Bytes that this process can still allocate: free on the card or held by the allocator, within the process's share.
+    (10 us, 90 behind a full queue; no synchronisation, and no launch that a capture would refuse.)"""
+    free, total = torch.cuda.mem_get_info(device)
     try:
-        return torch.empty_like(logits)
-    except torch.OutOfMemoryError:
-        return None
+        stats = torch.cuda.memory_stats_as_nested_dict(device)
+        held, used = (stats[f"{kind}_bytes"]["all"]["current"] for kind in ("reserved", "allocated"))
+    except (KeyError, RuntimeError):  # an allocator without statistics
+        return free
+    return min(free + held - used, int(total * torch.cuda.get_per_process_memory_fraction(device)) - used)
+
+
+class GradientRoom:
+    """Where the logits gradients of the head cross-entropies of one forward, ``calls`` of them, wait for its backward."""
+
+    def __init__(self, calls: int = 1):
+        self.calls = calls
+
+    def take(self, logits):
+        """The place for one, or None: it is made in the backward then, from the logits."""
+        left, self.calls = max(self.calls, 1), self.calls - 1
+        if left * logits.numel() * 2 > LABEL_GRADIENT_SHARE * _available_memory(logits.device):
+            return None
+        try:
+            return torch.empty_like(logits)
+        except torch.OutOfMemoryError:
+            return None
 
 
 # Whether the frozen-head cross-entropy takes its row statistics from the head product's epilogue
@@ -889,11 +911,12 @@ HEAD_CE_EPILOGUE_STATS = False
 
 def head_label_cross_entropy(x: torch.Tensor, weight: torch.Tensor, weight_t: torch.Tensor,
                              labels: torch.Tensor, ignore_index: int = -100,
-                             epilogue_stats: bool | None = None):
+                             epilogue_stats: bool | None = None, room: GradientRoom | None = None):
     """``logits = x @ weight.T`` and ``F.cross_entropy(logits, labels, ignore_index=...,
     reduction="none")`` (models/mtp/core.py:190-216) for a FROZEN ``weight [V, H]`` whose
     transpose ``weight_t [H, V]`` the caller keeps: returns ``(loss [...] f32, logits [..., V])``.
-    Gradient flows to ``x`` through the loss only; the returned logits are detached."""
+    Gradient flows to ``x`` through the loss only; the returned logits are detached.  ``room``: one for all calls of a forward
+    (None: this is the only one)."""
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight_t.dtype != torch.bfloat16:
         raise _lib.SpxError("head_label_cross_entropy takes bf16 operands")
     if weight.requires_grad:
@@ -906,8 +929,8 @@ def head_label_cross_entropy(x: torch.Tensor, weight: torch.Tensor, weight_t: to
     lab = labels.reshape(-1).to(torch.int64).contiguous()
     if epilogue_stats is None:
         epilogue_stats = HEAD_CE_EPILOGUE_STATS
-    loss, logits = _HeadLabelCE.apply(x2, weight, weight_t, lab, ignore_index, bool(epilogue_stats),
-                                      _label_one_pass(x2, weight, weight_t))
+    room = (room or GradientRoom()) if _label_one_pass(x2, weight) else None
+    loss, logits = _HeadLabelCE.apply(x2, weight, weight_t, lab, ignore_index, bool(epilogue_stats), room)
     return loss.view(labels.shape), logits.view(*labels.shape, weight.shape[0])
 
 

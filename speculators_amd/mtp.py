@@ -269,6 +269,7 @@ class MTPDraftModel(nn.Module):
         layer = self.mtp_layers[0]
 
         current = hidden_states
+        room = L.GradientRoom(steps)
         for step in range(steps):
             hid = current[:, :valid].reshape(1, b * valid, cfg.hidden_size)
             with torch.no_grad():
@@ -287,7 +288,7 @@ class MTPDraftModel(nn.Module):
                 # head + loss as one autograd node: the backward skips the ignored positions in the
                 # input-gradient product of the head (the returned logits carry no gradient)
                 unreduced, logits = L.head_label_cross_entropy(
-                    out.view(b, valid, cfg.hidden_size), head.w, head.wt, targets, IGNORE_INDEX)
+                    out.view(b, valid, cfg.hidden_size), head.w, head.wt, targets, IGNORE_INDEX, room=room)
             else:
                 logits = gemm.linear_staged(out, head, hip=True).view(b, valid, cfg.vocab_size)
                 unreduced = L.label_cross_entropy(logits, targets, IGNORE_INDEX)
