@@ -511,7 +511,7 @@ def head_terms_loss(loss_config, x, weight, weight_t, targets, d2t, target_stats
 
 
 LOSS_STEPS_MAX = 32            # SPX_LOSS_STEPS_MAX
-STEPS_LOGITS_BYTES = 1 << 32   # logits of several steps that are held at a time (at least one step's)
+STEPS_LOGITS_BYTES = 1 << 32   # logits of several steps that are held at a time (at least one step's; fewer where memory is short)
 
 
 class _HeadStepsLoss(torch.autograd.Function):
@@ -532,13 +532,22 @@ class _HeadStepsLoss(torch.autograd.Function):
         run.tokens = torch.empty(steps, t, device=dev, dtype=torch.int64)
         hits = torch.empty(steps, t, device=dev, dtype=torch.uint8)
         packed = torch.empty(steps * t, vocab, device=dev, dtype=torch.bfloat16) if grad else None
-        at_once = max(1, STEPS_LOGITS_BYTES // (2 * t * vocab))
-        for first in range(0, steps, at_once):
-            logits = [matmul_nt(x.reshape(t, x.shape[-1]), weight) for x in xs[first:first + at_once]]
+        at_once = min(steps, max(1, STEPS_LOGITS_BYTES // (2 * t * vocab)))
+        first = 0
+        while first < steps:
+            logits = None  # (freed before the next are made)
+            try:
+                logits = [matmul_nt(x.reshape(t, x.shape[-1]), weight) for x in xs[first:first + at_once]]
+            except torch.OutOfMemoryError:
+                if at_once == 1:
+                    raise
+                at_once //= 2
+                continue
             native.loss_steps_pass(run.op, run.terms, run.masked_first, run.mask, kind, run.targets, run.argmax, ints, floats,
                                    run.tokens, hits, packed, steps, first, *logits)
             if run.logits is not None:
                 run.logits += logits
+            first += len(logits)
         run.scalars, total = native.loss_steps_end(
             run.terms, run.mask, kind, run.prev, _lib.kind_code(run.prev) if run.prev is not None else 0, ints, floats, hits, steps,
             run.factor)
