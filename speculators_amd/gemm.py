@@ -152,7 +152,8 @@ def matmul_nt(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor | None = No
 def rows_graded(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor, row_of: torch.Tensor, row_weight: torch.Tensor,
                 scale: torch.Tensor, factor: float) -> torch.Tensor:
     """``matmul_nt(a, b, m_live)`` with row ``m`` multiplied by ``row_weight[row_of[m]] * (scale * factor)`` in fp32, before its
-    one rounding (``spx_gemm_bf16_rows_graded``)."""
+    one rounding (``spx_gemm_bf16_rows_graded``).  The parts that are chosen on the device, and with them the order of the fp32
+    sums, follow from the sizes and the row count alone, whatever product the workspace served before."""
     m, k = a.shape
     n = b.shape[0]
     if k != b.shape[1] or m_live.dtype != torch.int32 or row_of.dtype != torch.int32 or row_of.numel() < m:
@@ -168,7 +169,7 @@ def rows_graded(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor, row_of: 
     ws = _split_workspace(a.device, ws_numel) if ws_numel else None
     out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
     _lib.call("spx_gemm_bf16_rows_graded", a, a.stride(0), b, b.stride(0), out, n, m, n, k, m_live, row_of, row_weight, scale,
-              factor, TAIL_PARTS, parts, ws, ws.numel() * 4 if ws_numel else 0, _lib.stream_ptr(a.device))
+              factor, TAIL_PARTS, parts, ws, ws_numel * 4, _lib.stream_ptr(a.device))  # (the buffer may be larger: see above)
     return out
 
 
