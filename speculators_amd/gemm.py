@@ -31,9 +31,10 @@ if not 1 <= SPLIT_PARTS <= 8:
     raise ValueError(f"SPX_GEMM_SPLIT_PARTS must be 1 .. 8, got {SPLIT_PARTS}")
 
 
-# parts the last round's tiles of such a product with graded rows may be cut into, and partial tiles of 256 KB held for them
+# parts the last round's tiles of such a product with graded rows may be cut into (where SPX_GEMM_SPLIT_PARTS is set, it bounds
+# these, too), and partial tiles of 256 KB held for them
 # (22930 live rows x 151936 -> 2048: 208 tiles of a last round in 6 parts; with room for 1024 in one piece, 0.4 ms more of 10)
-LIVE_TAIL_PARTS, LIVE_TAIL_TILES = 8, 1280
+LIVE_TAIL_PARTS, LIVE_TAIL_TILES = SPLIT_PARTS if "SPX_GEMM_SPLIT_PARTS" in os.environ else 8, 1280
 # parts the tiles of a mostly empty last round of a product may be cut into (spx_gemm_bf16_nt_tail); 1 = never
 TAIL_PARTS = int(os.environ.get("SPX_GEMM_TAIL_PARTS", "4"))
 if not 1 <= TAIL_PARTS <= 8:

@@ -1,5 +1,9 @@
 """What the host hands to the graded live-row product (``gemm.rows_graded``): the workspace that its parts are chosen by."""
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -32,3 +36,12 @@ def test_workspace_is_the_one_asked_for(calls, m, n, k):
     gemm._split_workspace(torch.device("cpu"), 2 * alone[1] // 4 + 65536)  # left behind by a larger product
     assert calls(m, n, k) == alone
 
+
+
+@pytest.mark.parametrize("split,parts", [(None, 8), (1, 1), (2, 2), (3, 3), (4, 4), (8, 8)])
+def test_parts_are_bounded_by_the_variable(split, parts):
+    env = {k: v for k, v in os.environ.items() if k != "SPX_GEMM_SPLIT_PARTS"}
+    if split is not None:
+        env["SPX_GEMM_SPLIT_PARTS"] = str(split)
+    run = [sys.executable, "-c", "from speculators_amd import gemm; print(gemm.LIVE_TAIL_PARTS if gemm.SPLIT_PARTS > 1 else 1)"]
+    assert int(subprocess.run(run, env=env, check=True, capture_output=True, text=True).stdout) == parts
