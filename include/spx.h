@@ -830,6 +830,11 @@ int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void* b, int64_t
                               const float* scale, float factor, int32_t max_parts, int32_t split_parts, void* workspace,
                               int64_t workspace_bytes, void* stream);
 
+/* The parts that the call above cuts its contraction (on the 256 x 256 kernel: that of the last round of tiles) into for *m_live =
+ * live, with rows of c that 16-byte stores reach: what both its launches find. */
+int32_t spx_gemm_graded_parts(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts, int64_t workspace_bytes,
+                              int64_t live);
+
 /* The two ends of a packed-rows product (spx_*_bwd_packed -> spx_gemm_bf16_nt_rows).
  * spx_pack_row_map: row_map[r] = number of live rows before r if row r is live
  * (row_grad[r] != 0 and, when labels is not NULL, labels[r] != ignore_index), else -1;

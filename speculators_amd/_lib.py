@@ -152,6 +152,7 @@ SIGNATURES["spx_moe_sort_pairs"] = [_P, _I64, _I32, _I64, _P, _P, _P, _P, _P, _I
 SIGNATURES["spx_gemm_auto_workspace_bytes"] = [_I, _I64, _I64, _I64, _I32]
 SIGNATURES["spx_gemm_auto_us"] = [_I, _I64, _I64, _I64, _I32]
 SIGNATURES["spx_gemm_auto_tile"] = [_I, _I64, _I64, _I64, _I32]
+SIGNATURES["spx_gemm_graded_parts"] = [_I64, _I64, _I64, _I32, _I32, _I64, _I64]
 SIGNATURES["spx_gemm_bf16_auto_parts"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P]
 SIGNATURES["spx_gemm_bf16_auto"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P]
 SIGNATURES["spx_stage_upload"] = [_P, _I64, _P, _P, _I64, _I32, _P]

@@ -114,25 +114,27 @@ __host__ __device__ __forceinline__ void tail_plan(int n_tiles, int cus, int nsl
 // The same for a product whose rows are counted on the device, and for any last round: as many parts (at most max_parts, each
 // at least 16 slabs, tiles x parts at most `room` partial tiles) as make it shortest.  The times are those of the 256 x 256 tile,
 // as gemm_tile.hip has them, 16 us for a part's start and its 256 KB of partial results, and the pass behind it
-// (reduce_us there); one more part has to promise 3 %.  400 tiles: 256 whole ones, then 144 in 5 parts, 3 / 5 of a round in the
+// (reduce_us there); one more part has to promise 3 %.  In whole numbers, nanoseconds times compute units: the product, the pass
+// that adds its parts and the host each work the plan out, and have to find the same one however they are compiled.
+// 400 tiles: 256 whole ones, then 144 in 5 parts, 3 / 5 of a round in the
 // place of one.  x 32000, us, all tiles cut in up to 4 parts (where there are at most 512) / so: -> 4096, 6300 live of 9003 rows
 // 1455 / 1300, 4500 of them 1416 / 898, 4200 of 6000 1042 / 867; -> 8192, 2150 of 3072 1020 / 865; -> 2048, 1260 of 1800
 // 173 / 154, 900 of them 152 / 116, 1800 of them 202 / 208; worst 1800 of 3600 200 / 209.
-__device__ __forceinline__ void live_tail_plan(int n_tiles, int cus, int nslab, int max_parts, int room, int& first,
-                                               int& parts) {
+__host__ __device__ __forceinline__ void live_tail_plan(int n_tiles, int cus, int nslab, int max_parts, int room, int& first,
+                                                        int& parts) {
   first = n_tiles;
   parts = 1;
   const int rem = n_tiles > 0 ? n_tiles % cus : 0;
   if (rem == 0) return;
   auto rounds = [&](int wgs, int slabs) __attribute__((always_inline)) {
     const int last = wgs % cus;
-    return (float)slabs * ((float)(wgs / cus) * 1.41f + (last ? 1.18f + 0.23f * (float)last / (float)cus : 0.f));
+    return (int64_t)slabs * ((int64_t)(wgs / cus) * 1410 * cus + (last ? 1180 * cus + 230 * last : 0));
   };
-  float best = rounds(rem, nslab) + 6.9f;
+  int64_t best = rounds(rem, nslab) + 6900 * cus;
   for (int p = 2; p <= max_parts && nslab / p >= 16 && rem * p <= room; ++p) {
-    const float t = rounds(rem * p, (nslab + p - 1) / p) + 16.f * (float)((rem * p + cus - 1) / cus) + 4.1f +
-                    1.03e-6f * 65536.f * (float)(rem * p);
-    if (t < 0.97f * best) { best = t; first = n_tiles - rem; parts = p; }
+    const int64_t t = rounds(rem * p, (nslab + p - 1) / p) +
+                      (int64_t)cus * (16000 * ((rem * p + cus - 1) / cus) + 4100 + rem * p * 135 / 2);  // (67.5 ns a partial tile)
+    if (t * 100 < best * 97) { best = t; first = n_tiles - rem; parts = p; }
   }
 }
 
@@ -922,10 +924,24 @@ extern "C" int spx_gemm_bf16_nt_rows(const void* a, int64_t lda, const void* b, 
   return gemm_nt_impl(__func__, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream);
 }
 
+// partial tiles that fit
+static int graded_room(int64_t part_floats, int max_parts) {
+  return max_parts > 1 ? (int)std::min<int64_t>(part_floats / (kTM * kTN), 1 << 20) : 0;
+}
+
+int spx::nt_rows_graded_parts(int64_t live, int64_t N, int64_t K, int64_t part_floats, int max_parts) {
+  const int room = graded_room(part_floats, max_parts);
+  int first, parts = 1;
+  if (room)
+    live_tail_plan((int)((live + kTM - 1) / kTM * ((N + kTN - 1) / kTN)), compute_units(), (int)((K + kTK - 1) / kTK), max_parts, room,
+                   first, parts);
+  return parts;
+}
+
 int spx::nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                         int64_t M, int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws,
                         int64_t part_floats, int max_parts, void* stream) {
-  const int room = part_ws && max_parts > 1 ? (int)std::min<int64_t>(part_floats / (kTM * kTN), 1 << 20) : 0;
+  const int room = part_ws ? graded_room(part_floats, max_parts) : 0;
   return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, m_live, stream, nullptr, nullptr, 0, 0, room ? part_ws : nullptr,
                       room ? max_parts : 1, nullptr, 0, room, grade);
 }

@@ -184,21 +184,21 @@ struct Operand {
   }
 };
 
-// us of the pass that adds the parts of `partials` fp32 results in all
-__host__ __device__ __forceinline__ float reduce_us(float partials) { return 4.1f + 1.03e-6f * partials; }
-
 // The parts of a product whose rows are counted on the device: those that make it shortest, as the host has it for all M rows
-// (choose in gemm_tile.hip), for the tiles that are there.  max_parts = 0: as the host says.
+// (choose in gemm_tile.hip), for the tiles that are there.  max_parts = 0: as the host says.  In whole numbers, nanoseconds times
+// the workgroups that the chip holds: the product, the pass that adds its parts and the host each work the parts out, and have
+// to find the same however they are compiled.
 struct LiveCut {
   int max_parts, cap, slabs;  // cap: workgroups the chip holds
-  float s0, s1;               // of the tile's Config
-  __device__ __forceinline__ int parts(int tiles, float results) const {
+  int s0, s1;                 // of the tile's Config, in ns
+  __host__ __device__ __forceinline__ int parts(int tiles, int64_t results) const {
     int best = 1;
-    float us = 3.4e38f;
-    for (int n = 1; n <= max_parts && (n == 1 || tiles * n <= cap); ++n) {
-      const float t = (s0 + s1 * (float)min(tiles * n, cap) / (float)cap) * (float)((slabs + n - 1) / n) +
-                      (n > 1 ? reduce_us((float)n * results) : 0.f);
-      if (t < us) { us = t; best = n; }
+    int64_t ns = 0;
+    for (int n = 1; n <= max_parts && (n == 1 || (int64_t)tiles * n <= cap); ++n) {
+      const int wgs = tiles * n < cap ? tiles * n : cap;  // (n == 1: as many tiles as there are)
+      const int64_t t = ((int64_t)s0 * cap + (int64_t)s1 * wgs) * ((slabs + n - 1) / n) +
+                        (n > 1 ? cap * (4100 + n * results * 103 / 100000) : 0);
+      if (n == 1 || t < ns) { ns = t; best = n; }
     }
     return tiles > 0 ? best : 1;
   }
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   if (!AT && p.tile_tab) tiles_m = min(p.tile_tab[0], tiles_m);
   const int n_tiles = tiles_m * p.tiles_n;
   int parts = p.parts;
-  if (GRADE && p.cut.max_parts) parts = p.cut.parts(n_tiles, (float)M * (float)p.N);
+  if (GRADE && p.cut.max_parts) parts = p.cut.parts(n_tiles, (int64_t)M * p.N);
   const int n_wg = n_tiles * parts;
   if ((int)blockIdx.x >= n_wg) return;
   // one contiguous run of workgroups per XCD (they go to the eight XCDs round robin), tiles in it first, then parts:

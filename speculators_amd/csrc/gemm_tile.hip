@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restri
   const int M = m_live ? min(M_host, max(*m_live, 0)) : M_host;
   if (OUT == 0 && cut.max_parts) {
     const int tiles_m = (M + tm - 1) / tm;
-    parts = cut.parts(tiles_m * ((N + tn - 1) / tn), (float)M * (float)N);
+    parts = cut.parts(tiles_m * ((N + tn - 1) / tn), (int64_t)M * N);
     if (parts == 1) return;
     M_host = tiles_m * tm;
   }
@@ -285,6 +285,9 @@ struct Choice {
   float us;
 };
 
+// us of the pass that adds the parts of `partials` fp32 results in all
+static float reduce_us(float partials) { return 4.1f + 1.03e-6f * partials; }
+
 static float predict(const Config& c, int64_t tiles, int slabs) {
   const int64_t cap = (int64_t)kCus * c.per_cu, full = tiles / cap, rem = tiles % cap;
   float t = full * ((c.s0 + c.s1) * slabs + c.b);
@@ -336,6 +339,11 @@ static int64_t live_cut_floats(const Config& c, int64_t M, int64_t N, int64_t K,
   const int64_t tiles_n = (N + c.tn - 1) / c.tn, rows = (M + c.tm - 1) / c.tm * c.tm;
   if (tiles_n * 2 > kCus * c.per_cu) return 0;
   return std::min<int64_t>((int64_t)kCus * c.per_cu * c.tm * c.tn, kMaxParts * rows * N);
+}
+
+static LiveCut live_cut(const Config& c, int64_t K) {
+  const int slabs = (int)((K + kTK - 1) / kTK);
+  return {std::min(kMaxParts, slabs / kMinSlabs), kCus * c.per_cu, slabs, (int)(c.s0 * 1000.f + 0.5f), (int)(c.s1 * 1000.f + 0.5f)};
 }
 
 static Choice choose_tn(int64_t M, int64_t N, int64_t T, bool can_split) {
@@ -601,14 +609,23 @@ extern "C" int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void*
   // 768 of them 162 -> 93, 716 of 1024 98 -> 92, 512 of them 92 -> 69, 620 of 888 98 -> 90; -> 4096, 460 of 1536 345 -> 123; all rows
   // live: as before.
   const int64_t floats = tile::live_cut_floats(cfg, M, N, K, max_parts);
-  if (can_split(N) && vec && workspace && floats && workspace_bytes >= floats * (int64_t)sizeof(float)) {
-    const int slabs = (int)((K + tile::kTK - 1) / tile::kTK);
-    p.cut = {std::min(tile::kMaxParts, slabs / tile::kMinSlabs), tile::kCus * cfg.per_cu, slabs, cfg.s0, cfg.s1};
-  }
+  if (can_split(N) && vec && workspace && floats && workspace_bytes >= floats * (int64_t)sizeof(float)) p.cut = tile::live_cut(cfg, K);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (int rc = tile::launch_graded(fname, ch.tile, p, st)) return rc;
   if (ch.parts == 1 && !p.cut.max_parts) return SPX_OK;
   return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st, grade, p.cut, cfg.tm, cfg.tn);
+}
+
+extern "C" int32_t spx_gemm_graded_parts(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts,
+                                         int64_t workspace_bytes, int64_t live) {
+  if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1 || split_parts < 1) return 1;
+  const tile::Choice ch = tile::choose(2, M, N, K, max_parts, can_split(N) && workspace_bytes > 0);
+  live = std::min(std::max<int64_t>(live, 0), M);
+  if (ch.tile == tile::kBig) return nt_rows_graded_parts(live, N, K, workspace_bytes / (int64_t)sizeof(float), split_parts);
+  const tile::Config& cfg = tile::kNT[ch.tile];
+  const int64_t floats = tile::live_cut_floats(cfg, M, N, K, max_parts);
+  if (!can_split(N) || !floats || workspace_bytes < floats * (int64_t)sizeof(float)) return ch.parts;
+  return tile::live_cut(cfg, K).parts((int)((live + cfg.tm - 1) / cfg.tm * ((N + cfg.tn - 1) / cfg.tn)), live * N);
 }
 
 // ------------------------------------------------------------------------------------------ weight gradients

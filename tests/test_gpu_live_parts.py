@@ -65,3 +65,33 @@ def test_last_round_of_live_tiles_against_float64(n, live):
                       _lib.stream_ptr(a.device))
             assert (ws[room * 65536:] == 3).all() and (c[live:] == 2).all() and (c[:, n:] == 2).all()
             assert live == 0 or ((c[:live, :n].double() - want).abs() <= bound).all()
+
+
+# the 256 x 256 kernel (partial results a whole tile each), and the smaller tiles ([parts][whole tile rows][N])
+@pytest.mark.parametrize("m,n,k", [(5000, 4096, 4104), (1300, 2048, 8192), (513, 2048, 4096), (96, 64, 4096)])
+def test_device_and_host_find_the_same_parts(m, n, k):
+    from speculators_amd import _lib
+
+    lib = _lib.load()
+    tile = lib.spx_gemm_auto_tile(2, m, n, k, 4)
+    tm, tn = {0: (256, 256), 1: (128, 128), 2: (256, 128), 3: (64, 128)}[tile]
+    nbytes = lib.spx_gemm_auto_workspace_bytes(2, m, n, k, 4) if tile else 1024 << 18
+    a, b = torch.ones(m, k, device="cuda").bfloat16(), torch.ones(n, k, device="cuda").bfloat16()
+    order, weight = torch.arange(m, device="cuda", dtype=torch.int32), torch.ones(m, device="cuda")
+    found = set()
+    for live in sorted({1, tm, tm + 1, m // 3, m // 2, 2 * m // 3, m - 1, m}):
+        count = torch.tensor([live], dtype=torch.int32, device="cuda")
+        ws, c = torch.full((nbytes // 4,), 3.0, device="cuda"), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        _lib.call("spx_gemm_bf16_rows_graded", a, k, b, k, c, n, m, n, k, count, order, weight, torch.ones((), device="cuda"), 1.0,
+                  4, 8, ws, nbytes, _lib.stream_ptr(a.device))
+        parts = lib.spx_gemm_graded_parts(m, n, k, 4, 8, nbytes, live)
+        tile_rows = -(-live // tm)
+        one = tile_rows * -(-n // tn) % 256 * 65536 if tile == 0 else tile_rows * tm * n  # floats of one part
+        written = (ws != 3).nonzero()
+        assert (c[:live] == torch.tensor(float(k)).bfloat16().item()).all()
+        if parts == 1:
+            assert len(written) == 0
+        else:
+            assert (parts - 1) * one <= int(written[-1]) < parts * one
+        found.add(parts)
+    assert max(found) > 1  # (96 rows are cut in ten whatever counts)

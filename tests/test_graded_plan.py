@@ -1,4 +1,4 @@
-"""What the host hands to the graded live-row product (``gemm.rows_graded``): the workspace that its parts are chosen by."""
+"""The parts of the graded live-row product (``gemm.rows_graded``): the rule in exact arithmetic, and what the host hands over."""
 
 import os
 import subprocess
@@ -7,7 +7,7 @@ import sys
 import pytest
 import torch
 
-from speculators_amd import gemm
+from speculators_amd import _lib, gemm
 
 
 @pytest.fixture
@@ -45,3 +45,56 @@ def test_parts_are_bounded_by_the_variable(split, parts):
         env["SPX_GEMM_SPLIT_PARTS"] = str(split)
     run = [sys.executable, "-c", "from speculators_amd import gemm; print(gemm.LIVE_TAIL_PARTS if gemm.SPLIT_PARTS > 1 else 1)"]
     assert int(subprocess.run(run, env=env, check=True, capture_output=True, text=True).stdout) == parts
+
+
+def _rounds(wgs, slabs, cus=256):
+    last = wgs % cus
+    return slabs * (wgs // cus * 1410 * cus + (1180 * cus + 230 * last if last else 0))
+
+
+def _last_round(tiles, slabs, max_parts, room, cus=256):
+    """Parts of the tiles of the last round: the fewest nanoseconds, each further part 3 % less."""
+    rem, parts = tiles % cus, 1
+    best = _rounds(rem, slabs) + 6900 * cus
+    for p in range(2, max_parts + 1):
+        if rem == 0 or slabs // p < 16 or rem * p > room:
+            break
+        t = _rounds(rem * p, -(-slabs // p)) + cus * (16000 * -(-rem * p // cus) + 4100 + rem * p * 135 // 2)
+        if t * 100 < best * 97:
+            best, parts = t, p
+    return parts
+
+
+def _small_tiles(tiles, results, slabs, s0, s1, cap):
+    """Parts of a product on the smaller tiles: the fewest nanoseconds of those that fit the chip at once."""
+    def ns(n):
+        return (s0 * cap + s1 * min(tiles * n, cap)) * -(-slabs // n) + (cap * (4100 + n * results * 103 // 100000) if n > 1 else 0)
+
+    fit = [n for n in range(1, min(12, slabs // 6) + 1) if n == 1 or tiles * n <= cap]
+    return min(fit, key=ns) if tiles else 1
+
+
+@pytest.mark.parametrize("m,n,k", [(9003, 4096, 32000), (32760, 2048, 151936), (70000, 256, 4104)])
+@pytest.mark.parametrize("room", [0, 100, 1024, 2040])
+@pytest.mark.parametrize("split", [1, 3, 8])
+def test_parts_of_the_last_round(m, n, k, room, split):
+    lib = _lib.load()
+    assert lib.spx_gemm_auto_tile(2, m, n, k, 4) == 0
+    for tile_rows in range(-(-m // 256) + 1):
+        want = _last_round(tile_rows * -(-n // 256), -(-k // 64), split, room if split > 1 else 0)
+        for live in {max(0, tile_rows * 256 - 255), tile_rows * 256}:
+            assert lib.spx_gemm_graded_parts(m, n, k, 4, split, room * 262144, live) == want, live
+
+
+TILES = {1: (128, 128, 1, 350, 140), 2: (256, 128, 1, 520, 250), 3: (64, 128, 2, 180, 420)}  # rows, columns, per unit, ns
+
+
+@pytest.mark.parametrize("tile,m,n,k", [(1, 513, 2048, 4096), (2, 1300, 2048, 8192), (3, 96, 64, 4096), (2, 1536, 2048, 32000)])
+def test_parts_on_the_smaller_tiles(tile, m, n, k):
+    lib = _lib.load()
+    assert lib.spx_gemm_auto_tile(2, m, n, k, 4) == tile
+    tm, tn, per, s0, s1 = TILES[tile]
+    nbytes = lib.spx_gemm_auto_workspace_bytes(2, m, n, k, 4)
+    for live in [0, 1, *range(tm - 1, m, tm), *range(tm, m, tm), m]:
+        want = _small_tiles(-(-live // tm) * -(-n // tn), live * n, -(-k // 64), s0, s1, 256 * per)
+        assert lib.spx_gemm_graded_parts(m, n, k, 4, 8, nbytes, live) == want, live
