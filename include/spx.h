@@ -830,6 +830,9 @@ int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void* b, int64_t
                               const float* scale, float factor, int32_t max_parts, int32_t split_parts, void* workspace,
                               int64_t workspace_bytes, void* stream);
 
+/* What the call above can use of a workspace, for any *m_live up to M: the parts of its last round (at most 8 x 256 tiles of
+ * 256 KB, 0.5 GB) or those of the smaller tiles; more changes nothing. */
+int64_t spx_gemm_graded_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts);
 /* The parts that the call above cuts its contraction (on the 256 x 256 kernel: that of the last round of tiles) into for *m_live =
  * live, with rows of c that 16-byte stores reach: what both its launches find. */
 int32_t spx_gemm_graded_parts(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts, int64_t workspace_bytes,

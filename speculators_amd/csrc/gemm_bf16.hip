@@ -929,6 +929,19 @@ static int graded_room(int64_t part_floats, int max_parts) {
   return max_parts > 1 ? (int)std::min<int64_t>(part_floats / (kTM * kTN), 1 << 20) : 0;
 }
 
+int64_t spx::nt_rows_graded_floats(int64_t M, int64_t N, int64_t K, int max_parts) {
+  if (max_parts <= 1) return 0;
+  const int cus = compute_units(), nslab = (int)((K + kTK - 1) / kTK);
+  const int64_t tiles_n = (N + kTN - 1) / kTN, rows = (M + kTM - 1) / kTM;
+  int64_t most = 0;
+  for (int64_t r = 1; r <= std::min<int64_t>(rows, cus); ++r) {  // (the last rounds repeat behind as many tile rows)
+    int first, parts, rem = (int)(r * tiles_n % cus);
+    live_tail_plan(rem, cus, nslab, max_parts, cus * max_parts, first, parts);
+    if (parts > 1) most = std::max<int64_t>(most, (int64_t)rem * parts);
+  }
+  return most * kTM * kTN;
+}
+
 int spx::nt_rows_graded_parts(int64_t live, int64_t N, int64_t K, int64_t part_floats, int max_parts) {
   const int room = graded_room(part_floats, max_parts);
   int first, parts = 1;

@@ -616,6 +616,13 @@ extern "C" int spx_gemm_bf16_rows_graded(const void* a, int64_t lda, const void*
   return tile::launch_reduce<0>(fname, p.part_ws, c, ldc, M, N, ch.parts, m_live, st, grade, p.cut, cfg.tm, cfg.tn);
 }
 
+extern "C" int64_t spx_gemm_graded_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts) {
+  if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1 || split_parts < 1) return 0;
+  if (tile::choose(2, M, N, K, max_parts, can_split(N)).tile != tile::kBig)
+    return spx_gemm_auto_workspace_bytes(2, M, N, K, max_parts);
+  return nt_rows_graded_floats(M, N, K, std::min(split_parts, 8)) * (int64_t)sizeof(float);
+}
+
 extern "C" int32_t spx_gemm_graded_parts(int64_t M, int64_t N, int64_t K, int32_t max_parts, int32_t split_parts,
                                          int64_t workspace_bytes, int64_t live) {
   if (M <= 0 || N <= 0 || K <= 0 || max_parts < 1 || split_parts < 1) return 1;

@@ -20,6 +20,8 @@ struct RowGrade {
 int nt_rows_graded(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
                    int64_t N, int64_t K, const int32_t* m_live, const RowGrade& grade, float* part_ws, int64_t part_floats,
                    int max_parts, void* stream);
+// the most floats of part_ws that it uses for any number of rows up to M
+int64_t nt_rows_graded_floats(int64_t M, int64_t N, int64_t K, int max_parts);
 // the parts of its last round of tiles for `live` rows
 int nt_rows_graded_parts(int64_t live, int64_t N, int64_t K, int64_t part_floats, int max_parts);
 

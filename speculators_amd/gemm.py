@@ -31,10 +31,9 @@ if not 1 <= SPLIT_PARTS <= 8:
     raise ValueError(f"SPX_GEMM_SPLIT_PARTS must be 1 .. 8, got {SPLIT_PARTS}")
 
 
-# parts the last round's tiles of such a product with graded rows may be cut into (where SPX_GEMM_SPLIT_PARTS is set, it bounds
-# these, too), and partial tiles of 256 KB held for them
-# (22930 live rows x 151936 -> 2048: 208 tiles of a last round in 6 parts; with room for 1024 in one piece, 0.4 ms more of 10)
-LIVE_TAIL_PARTS, LIVE_TAIL_TILES = SPLIT_PARTS if "SPX_GEMM_SPLIT_PARTS" in os.environ else 8, 1280
+# parts the last round's tiles of such a product with graded rows may be cut into; where SPX_GEMM_SPLIT_PARTS is set, it bounds
+# these, too
+LIVE_TAIL_PARTS = SPLIT_PARTS if "SPX_GEMM_SPLIT_PARTS" in os.environ else 8
 # parts the tiles of a mostly empty last round of a product may be cut into (spx_gemm_bf16_nt_tail); 1 = never
 TAIL_PARTS = int(os.environ.get("SPX_GEMM_TAIL_PARTS", "4"))
 if not 1 <= TAIL_PARTS <= 8:
@@ -125,6 +124,14 @@ def _plan(form: int, m: int, n: int, k: int, parts: int):
             lib.spx_gemm_auto_us(form, m, n, k, parts))
 
 
+@functools.lru_cache(maxsize=4096)
+def _graded_workspace(m: int, n: int, k: int, parts: int, split: int) -> int:
+    """Workspace elements of ``spx_gemm_bf16_rows_graded``: all that it can use for any number of rows that count, up to 0.5 GB.
+    (x 151936 -> 2048, room for 1280 partial tiles / so: 216 tiles in the last round whole 3592 us, in 7 parts 3438, 224 whole
+    3625, in 8 parts 3507; behind a whole round 7210 / 7016 and 7213 / 7078; x 128256, 216 tiles 3055 / 2940.)"""
+    return _lib.load().spx_gemm_graded_workspace_bytes(m, n, k, parts, split) // 4
+
+
 # how a product runs, as csrc/layer_host.cpp numbers it: on spx_gemm_bf16_auto (NT or NN form), on the 256 x 256 kernel
 # without or with its last round cut, or in the library
 AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL = range(6)
@@ -163,10 +170,8 @@ def rows_graded(a: torch.Tensor, b: torch.Tensor, m_live: torch.Tensor, row_of: 
         raise ValueError("row weights and scale are contiguous fp32")
     if b.stride(1) != 1:
         b = b.contiguous()
-    big, ws_numel, _ = _plan(2, m, n, k, TAIL_PARTS)
     parts = LIVE_TAIL_PARTS if SPLIT_PARTS > 1 else 1
-    if big:
-        ws_numel = min(LIVE_TAIL_TILES, parts * -(-m // 256) * -(-n // 256)) * 65536 if parts > 1 and k >= 64 * 16 * 2 else 0
+    ws_numel = _graded_workspace(m, n, k, TAIL_PARTS, parts)
     ws = _split_workspace(a.device, ws_numel) if ws_numel else None
     out = torch.empty(m, n, device=a.device, dtype=torch.bfloat16)
     _lib.call("spx_gemm_bf16_rows_graded", a, a.stride(0), b, b.stride(0), out, n, m, n, k, m_live, row_of, row_weight, scale,

@@ -98,3 +98,20 @@ def test_parts_on_the_smaller_tiles(tile, m, n, k):
     for live in [0, 1, *range(tm - 1, m, tm), *range(tm, m, tm), m]:
         want = _small_tiles(-(-live // tm) * -(-n // tn), live * n, -(-k // 64), s0, s1, 256 * per)
         assert lib.spx_gemm_graded_parts(m, n, k, 4, 8, nbytes, live) == want, live
+
+
+# as many partial tiles as the plan asks for at any number of rows: few rows, whole rounds only, every last round there is
+@pytest.mark.parametrize("m,n,k", [(3001, 4096, 32000), (9003, 4096, 32000), (32760, 2048, 151936), (70000, 256, 4104),
+                                   (5000, 65536, 8192), (5000, 8192, 56)])
+@pytest.mark.parametrize("split", [1, 3, 8])
+def test_workspace_holds_the_parts_of_any_row_count(m, n, k, split):
+    lib = _lib.load()
+    assert lib.spx_gemm_auto_tile(2, m, n, k, 4) == 0
+    most = 0
+    for tile_rows in range(1, -(-m // 256) + 1):
+        tiles = tile_rows * -(-n // 256)
+        parts = _last_round(tiles, -(-k // 64), split, 256 * 8)
+        most = max(most, tiles % 256 * parts if parts > 1 else 0)
+    nbytes = lib.spx_gemm_graded_workspace_bytes(m, n, k, 4, split)
+    assert nbytes == most * 262144
+    assert gemm._graded_workspace(m, n, k, 4, split) * 4 == nbytes
