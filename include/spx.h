@@ -979,8 +979,9 @@ int spx_moe_sort_pairs(const int64_t* idx, int64_t tokens, int32_t k, int64_t ex
  *                         outside [0, src_rows) gives a zero row)
  *   spx_moe_combine_rows: out[t] = sum_j weight[t, j] * sorted[pos[t, j]], j = 0 .. k-1 in that
  *                         order in fp32, one rounding (weight f32 [tokens, k] or NULL = ones)
- *   spx_moe_pair_dot:     out[t, j] = <a[t], sorted[pos[t, j]]> in fp32 (the gradient of the
- *                         routing weights). */
+ *   spx_moe_pair_dot:     out[t, j] = <a[t], sorted[pos[t, j]]> in fp32 (the gradient of the routing weights from
+ *                         the experts' output rows, for a caller that keeps them; spx_moe_swiglu_bwd has it
+ *                         from the activations). */
 int spx_moe_gather_rows(const void* x, int64_t ld_x, int64_t src_rows, const int32_t* src_row,
                         const float* scale, void* out, int64_t ld_out, int64_t rows, int64_t H,
                         void* stream);

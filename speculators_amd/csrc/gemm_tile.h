@@ -347,8 +347,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
     if (f < kMI) fa[set][f] = OA::read(a_rd, rd, wm, f, kk, lane);
     else fb[set][f - kMI] = OB::read(b_rd, rd, wn, f - kMI, kk, lane);
   };
-  // Grouped NT and NN: a wave whose rows are all past its group's loads and waits with the others, but reads and multiplies
-  // nothing: a group of 80 rows on average is half a tile.  4096 tokens, top 10 of 512 experts of uneven popularity, gate/up 470
+  // Grouped NT and NN: a wave whose rows are all past its group's loads and waits with the others, but multiplies nothing
+  // (nor reads its operands, where there are several slab buffers): a group of 80 rows on average is half a tile.  4096 tokens, top 10 of 512 experts of uneven popularity, gate/up 470
   // -> 448 us, down 256 -> 248, its input gradient 227 -> 226, gate/up's 425 -> 416; 12000 tokens 685 -> 676, 409 -> 402, 342 -> 341, 725 -> 695;
   // 80 rows each: no difference.
   constexpr bool kSkip = !AT && STREAM;

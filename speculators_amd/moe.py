@@ -115,62 +115,6 @@ def gemm_tn_grouped_multi(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tenso
     return out
 
 
-class _ExpertStacks:
-    """Inputs, output gradients and group boundaries of all uses of one expert weight stack in one
-    forward / backward, one use below the other, so that the stack's weight gradient is ONE
-    multi-segment grouped product when autograd reaches its staging node (the sum over the uses
-    happens in the MFMA accumulators and the gradient is written once)."""
-
-    def __init__(self, staged: Staged, rows: int, x_cols: int, dy_cols: int):
-        w = staged.w
-        # (no reference back to `staged`: it owns this object and its hook, and the buffers go
-        # with it as soon as the graph is dropped)
-        self.w_shape, self.rows, self.dy_cols = w.shape, rows, dy_cols
-        self.x = torch.empty(staged.uses * rows, x_cols, device=w.device, dtype=torch.bfloat16)
-        self.dy = None
-        self.off = torch.zeros(staged.uses, w.shape[0] + 1, device=w.device, dtype=torch.int32)
-        self.fill = 0
-        self.live = False
-        staged._finishers.append(self.add_gradient)
-
-    @staticmethod
-    def use(staged: Staged, rows: int, x_cols: int, dy_cols: int):
-        """``(stacks, use index)`` for the next product against ``staged``, or ``(None, -1)`` when
-        there is nothing to gain (frozen, one use, no graph) or no room."""
-        if staged.token is None or staged.uses <= 1 or not torch.is_grad_enabled():
-            return None, -1
-        st = staged.aux
-        if st is None:
-            st = staged.aux = _ExpertStacks(staged, rows, x_cols, dy_cols)
-        if st.rows != rows or st.fill >= staged.uses:
-            return None, -1
-        st.fill += 1
-        return st, st.fill - 1
-
-    def x_slot(self, u: int) -> torch.Tensor:
-        return self.x[u * self.rows:(u + 1) * self.rows]
-
-    def dy_slot(self, u: int) -> torch.Tensor:
-        if self.dy is None:
-            self.dy = torch.empty(self.x.shape[0], self.dy_cols, device=self.x.device, dtype=torch.bfloat16)
-        return self.dy[u * self.rows:(u + 1) * self.rows]
-
-    def record(self, u: int, offsets: torch.Tensor):
-        self.off[u].copy_(offsets)
-        self.live = True
-
-    def add_gradient(self, acc, dtype=torch.float32):
-        if not self.live:
-            return acc
-        fresh = acc is None
-        if fresh:
-            acc = torch.empty(self.w_shape, device=self.x.device, dtype=dtype)
-        gemm_tn_grouped_multi(self.dy, self.x, self.off, acc, accumulate=not fresh)
-        self.off.zero_()  # uses whose backward does not run next time contribute nothing
-        self.live = False
-        return acc
-
-
 def gather_rows(x2: torch.Tensor, src_row: torch.Tensor, scale: torch.Tensor | None = None,
                 out: torch.Tensor | None = None) -> torch.Tensor:
     """``out[p] = scale[p] * x2[src_row[p]]`` (bf16 rows, ``src_row`` int32, ``scale`` fp32)."""
@@ -314,19 +258,15 @@ class _ExpertsMLP(torch.autograd.Function):
         w_gu, w_dn = st_gu.w, st_dn.w  # [E, 2I, H], [E, H, I]
         st_gu.applied += 1
         st_dn.applied += 1
-        e, i2, h = w_gu.shape
+        e, i2, _ = w_gu.shape
         inter = i2 // 2
         order, src_row, pos, off = sort_pairs(idx, e)
         rows = src_row.numel()
         st = _lib.stream_ptr(x2.device)
-        # with several uses per forward the products' inputs (the down projection's: in the backward) go straight into
-        # the stacks that the one weight-gradient product over all uses reads
-        stack_gu, use_gu = _ExpertStacks.use(st_gu, rows, h, i2)
-        stack_dn, use_dn = _ExpertStacks.use(st_dn, rows, inter, h)
         picked = None
         if x2.stride(1) != 1:
             x2 = x2.contiguous()
-        if stack_gu is None and stack_dn is None and _Picked.takes(x2, rows, e):
+        if _Picked.takes(x2, rows, e):
             # (the products' 32-bit offsets span the rows as they lie: of a column slice of a wide buffer, a copy is picked;
             # and one where the backward reads the tokens, which the caller may write to by then: 4096 x 2048 14 us of 2296,
             # 18 on torch's clone)
@@ -337,7 +277,7 @@ class _ExpertsMLP(torch.autograd.Function):
             if not ctx.needs_input_grad[3]:
                 xs = None
         else:
-            xs = gather_rows(x2, src_row, out=None if stack_gu is None else stack_gu.x_slot(use_gu))
+            xs = gather_rows(x2, src_row)
             hid = gemm_nt_grouped(xs, w_gu, off)
         act = torch.empty(rows, inter, device=x2.device, dtype=torch.bfloat16)
         up = hid[:, inter:]
@@ -349,7 +289,6 @@ class _ExpertsMLP(torch.autograd.Function):
         ctx.save_for_backward(xs, hid, pos, src_row, off, order, wts)
         ctx.picked = picked
         ctx.staged = (st_gu, st_dn)
-        ctx.stacks = ((stack_gu, use_gu), (stack_dn, use_dn))
         ctx.score_dtype = scores.dtype
         return out
 
@@ -361,21 +300,16 @@ class _ExpertsMLP(torch.autograd.Function):
         inter = i2 // 2
         dout = dout.to(torch.bfloat16).contiguous()
         st = _lib.stream_ptr(dout.device)
-        (stack_gu, use_gu), (stack_dn, use_dn) = ctx.stacks
         want_gu, want_dn = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
         picked = ctx.picked
         if picked is not None:
             dys = dout
             dact = picked.rows_of(1, dout, st_dn.w, True)
         else:
-            dys = gather_rows(dout, src_row, out=stack_dn.dy_slot(use_dn) if stack_dn is not None and want_dn else None)
+            dys = gather_rows(dout, src_row)
             dact = gemm_nn_grouped(dys, st_dn.w, off)
-        dh = (stack_gu.dy_slot(use_gu) if stack_gu is not None and want_gu
-              else torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16))
-        act = None
-        if want_dn:
-            act = (torch.empty(rows, inter, device=dout.device, dtype=torch.bfloat16) if stack_dn is None
-                   else stack_dn.x_slot(use_dn))
+        dh = torch.empty(rows, i2, device=dout.device, dtype=torch.bfloat16)
+        act = torch.empty(rows, inter, device=dout.device, dtype=torch.bfloat16) if want_dn else None
         dscores = None
         if ctx.needs_input_grad[1]:
             dscores = torch.empty(wts.shape, device=dout.device, dtype=ctx.score_dtype if ctx.score_dtype == torch.bfloat16
@@ -386,18 +320,14 @@ class _ExpertsMLP(torch.autograd.Function):
         # for 40960 rows) and are read out of the memory-side cache, which the input gradient's pass over the weights (2.1 GB)
         # would leave empty.  4096 tokens, top 10 of 512 experts: 621 + 322 -> 537 + 276 us, the pass 2458 -> 2310.
         marks = {}
-        for need, staged, dy2, x2, stack, use, tokens in ((want_dn, st_dn, dys, act, stack_dn, use_dn, 0),
-                                                         (want_gu, st_gu, dh, xs, stack_gu, use_gu, 1)):
+        for need, staged, dy2, x2, tokens in ((want_dn, st_dn, dys, act, 0), (want_gu, st_gu, dh, xs, 1)):
             if not need:
                 continue
-            if stack is not None:
-                stack.record(use, off)  # the product runs once, over all uses, in the staging node
+            buf, holds = staged.grad_buffer()
+            if picked is not None:
+                picked.weight_gradient(dy2, x2, tokens, buf, holds)
             else:
-                buf, holds = staged.grad_buffer()
-                if picked is not None:
-                    picked.weight_gradient(dy2, x2, tokens, buf, holds)
-                else:
-                    gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
+                gemm_tn_grouped(dy2, x2, off, buf, accumulate=holds)
             marks[staged] = staged.mark()
         dx = None
         if ctx.needs_input_grad[0]:

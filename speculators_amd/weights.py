@@ -155,7 +155,7 @@ class Staged:
     is expected to run against it (the size of the input / output-gradient buffers)."""
 
     __slots__ = ("w", "token", "rows_of", "uses", "_wt", "_xs", "_fill", "_dys", "_live", "_extras",
-                 "_marked", "_acc", "aux", "_finishers", "_task", "applied", "bf16_params")
+                 "_marked", "_acc", "_task", "applied", "bf16_params")
 
     def __init__(self, w, rows_of, uses: int = 1, bf16_params: bool = False):
         self.w = w
@@ -172,8 +172,6 @@ class Staged:
         self._acc = None   # gradient buffer of uses that add their gradient themselves
         self.applied = 0   # products of this forward whose gradient goes to that buffer
         self.bf16_params = bf16_params  # the parameters are bf16: a gradient written once may be bf16 itself
-        self.aux = None    # whatever a family of products keeps per staged weight (the expert stacks)
-        self._finishers = []  # callables (acc, dtype of a fresh acc) -> acc that add deferred gradients at the end
         self._task = None     # the backward pass (autograd graph task) the recorded uses belong to
 
     @property
@@ -287,7 +285,7 @@ class Staged:
                 runs[-1][1] += n
             else:
                 runs.append([r0, n])
-        if bf16_ok and acc is None and len(runs) == 1 and not self._extras and not self._finishers:
+        if bf16_ok and acc is None and len(runs) == 1 and not self._extras:
             r0, n = runs[0]
             dy, x = self._dys[r0:r0 + n], self._xs[r0:r0 + n]
             if _tn_ok(dy) and _tn_ok(x):
@@ -295,7 +293,7 @@ class Staged:
 
                 self._dys, self._live, self._marked = None, [], False
                 return gemm_tn(dy, x, out_dtype=torch.bfloat16)
-        if bf16_ok and acc is None and not runs and len(self._extras) == 1 and not self._finishers:
+        if bf16_ok and acc is None and not runs and len(self._extras) == 1:
             dy, x = self._extras[0]
             if _tn_ok(dy) and _tn_ok(x):
                 from .gemm import gemm_tn
@@ -306,10 +304,6 @@ class Staged:
             acc = wgrad_product(self._dys[r0:r0 + n], self._xs[r0:r0 + n], acc)
         for dy2, x2 in self._extras:
             acc = wgrad_product(dy2, x2, acc)
-        last = len(self._finishers) - 1
-        for i, add_deferred in enumerate(self._finishers):
-            # (a gradient that is one product writes bf16 itself, as above)
-            acc = add_deferred(acc, torch.bfloat16 if bf16_ok and i == last else torch.float32)
         self._dys, self._live, self._extras, self._marked, self._acc = None, [], [], False, None
         return acc
 
