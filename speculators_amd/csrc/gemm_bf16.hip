@@ -13,13 +13,19 @@
 // (lane i -> byte 16 i), so every fetch is a whole 128-byte line; the
 // bank-conflict-free layout comes from WHICH 16-byte K chunk a lane fetches:
 // chunk c of row r sits in slot c ^ f(r), f(r) = (r & 7) ^ ((r >> 3) & 1).
-// Two slab buffers: the loads of slab s+1 are in flight while slab s is
-// multiplied.  They are issued one at a time between the MFMAs (a burst would
-// stall the wave at issue until the memory pipeline has room), and so are the
-// LDS reads: operand fragments are double buffered in registers, the reads of
+// The loads of slab s+2 are issued while slab s is multiplied, one at a time between the
+// MFMAs (a burst would stall the wave at issue until the memory pipeline has room), and so
+// are the LDS reads: operand fragments are double buffered in registers, the reads of
 // K step kk+1 (32 columns) run under the MFMAs of step kk, and the last step of a
 // slab is multiplied after the barrier that opens the next slab, so no LDS latency
 // is exposed and there is one barrier per slab.
+// Two slab buffers of A and three of B, all the LDS there is.  B of slab s+2 goes into the third while
+// slab s is still being read, A into the buffer that the barrier inside slab s frees: so the 16 loads
+// of a slab follow each other evenly, one per eight MFMAs, and each has 64 to 192 MFMAs to land.
+// With two buffers of each all 16 had to follow that barrier, one per four MFMAs, to have 64 left; where
+// each of them takes the wave's issue for longer than an MFMA takes the matrix pipe, that left the pipe waiting.
+// Before / now, us: 4096 x 4096 -> 32000 778 / 741, 4096 x 14336 -> 4096 324 / 305, 20013 x 32000 -> 4096
+// 3741 / 3383 (1550 TFLOP/s), 32760 x 2048 -> 12288 1368 / 1276, 512 x 2048 -> 32000 53.4 / 52.
 //
 // The accumulators are kept transposed (lane = row of C, registers = 4
 // consecutive columns); v_permlane16_swap pairs them into 8 consecutive
@@ -40,6 +46,8 @@ namespace spx {
 #define SPX_GEMM_WN 2
 #define SPX_GEMM_MINW 1
 #define SPX_GEMM_READ_EVERY 2  // MFMAs per LDS fragment read
+#define SPX_GEMM_LOAD_EVERY 8  // MFMAs per global -> LDS load ...
+#define SPX_GEMM_LOAD_AT 2     // ... of which the load follows this one (the reads follow the odd ones)
 constexpr int kWM = SPX_GEMM_WM, kWN = SPX_GEMM_WN;  // waves along M / N of the tile
 constexpr int kNW = kWM * kWN;
 constexpr int kGemmThreads = 64 * kNW;
@@ -50,7 +58,7 @@ constexpr int kRowBytes = kTK * 2;                          // 128
 constexpr int kABytes = kTM * kRowBytes;                    // one slab of A: 32 KB
 constexpr int kBBytes = kTN * kRowBytes;
 constexpr int kBBase = 2 * kABytes;
-constexpr int kGemmSmem = 2 * (kABytes + kBBytes);  // 128 KB
+constexpr int kGemmSmem = 2 * kABytes + 3 * kBBytes;  // 160 KB: all there is
 constexpr int kLA = kTM / 8 / kNW;                  // wave-loads of A per wave per slab
 constexpr int kLB = kTN / 8 / kNW;
 constexpr int kL = kLA + kLB;
@@ -288,16 +296,17 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   const uint32_t lds_a = lds0 + wave * (8 * kLA) * kRowBytes;
   const uint32_t lds_b = lds0 + kBBase + wave * (8 * kLB) * kRowBytes;
 
-  uint32_t bufoff = 0;  // slab buffer the next loads go to
-  int ld_k0 = 0;        // first K column of the slab being loaded
-  // load l (A loads first, then B) of the slab at ld_k0; full: the slab lies inside K
+  uint32_t buf_a = 0, buf_b = 0;  // slab buffers the next loads go to
+  int k_a = 0, k_b = 0;           // first K column of the slabs being loaded
+  // load l (A loads first, then B) of the slabs at k_a, k_b; full: they lie inside K
   auto issue_one = [&](int l, bool full) __attribute__((always_inline)) {
     const bool isa = l < kLA;
     const int j = isa ? l : l - kLA;
     int voff = isa ? aoff[j] : boff[j];
+    const int ld_k0 = isa ? k_a : k_b;
     if (!full) voff = (ld_k0 + gchunk[j & 1] * 8 < K) ? voff : kOob;
     const u32x4 res = isa ? ares : bres;
-    const uint32_t base = (isa ? lds_a : lds_b) + bufoff;
+    const uint32_t base = isa ? lds_a + buf_a : lds_b + buf_b;
     if (kImm) {
       const uint32_t grp = base + (j & ~3) * 8 * kRowBytes;
       switch (j & 3) {
@@ -310,17 +319,19 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
       load_to_lds16<0>(res, base + j * 8 * kRowBytes, voff, ld_k0 * 2);
     }
   };
-  auto next_slab = [&]() __attribute__((always_inline)) { bufoff ^= kABytes; ld_k0 += kTK; };
+  auto next_a = [&]() __attribute__((always_inline)) { buf_a ^= kABytes; k_a += kTK; };
+  auto next_b = [&]() __attribute__((always_inline)) { buf_b = buf_b == 2 * kBBytes ? 0 : buf_b + kBBytes; k_b += kTK; };
 
   // read side: row = lane % 16 of a 16-row block, K chunk 4 kk + lane / 16 in slot chunk ^ f(row)
   const int fr = (r16 & 7) ^ (r16 >> 3);
   const int off0 = r16 * kRowBytes + ((q ^ fr) * 16);
-  uint32_t a_rd[kKSteps], b_rd[kKSteps];  // per K step of 32; bit 15 selects the slab buffer
+  uint32_t a_rd[kKSteps], b_rd[kKSteps], b_rd0[kKSteps];  // per K step of 32; bit 15 selects the slab buffer of A
 #pragma unroll
   for (int kk = 0; kk < kKSteps; ++kk) {
     a_rd[kk] = wm * kRowBytes + (off0 ^ (kk * 64));
-    b_rd[kk] = kBBase + wn * kRowBytes + (off0 ^ (kk * 64));
+    b_rd0[kk] = b_rd[kk] = kBBase + wn * kRowBytes + (off0 ^ (kk * 64));
   }
+  uint32_t rd_b = 0;  // slab buffer of B that is read
 
   bf16x8 fa[2][kMI], fb[2][kNI];
   // operand fragment f (A fragments first, then B) of K step kk into register set `set`
@@ -349,45 +360,50 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
           read_one(set ^ 1, rk, reads++);
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (nl > 0 && (nl >= kN || idx % (kN / nl) == kN / nl - 1) && loads < nl) {
+        if (loads < nl && idx % SPX_GEMM_LOAD_EVERY == SPX_GEMM_LOAD_AT) {
           issue_one(l0 + loads++, full);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
   };
 
-  // the loads of a slab are issued in the step after the barrier that frees its buffer, one per
-  // four MFMAs; the step after that gives them time to land
   static_assert(kKSteps == 2, "a slab is two K steps: one before, one after the barrier");
-  constexpr int kLdT = kL;
   // one slab: on entry set 0 holds (or is receiving) K step 0 of slab s and the loads of slab s+1
   // are issued
   auto slab = [&](bool full) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    step(0, 1, 0, 0, full);
-    next_slab();
-    // every read of this slab's buffer has returned once set 1 is complete; then the
-    // barrier says: slab s+1 has landed for everybody, this buffer is free
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // K step 0 of slab s, under it the reads of step 1 and the loads of B of slab s+2
+    step(0, 1, kLA, kLB, full);
+    next_b();
+    // every read of this slab's buffers has returned once set 1 is complete; then the
+    // barrier says: slab s+1 has landed for everybody, these buffers are free
+    static_assert(kLB == 8, "the loads of B of slab s+2 may be on their way");
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
+    rd_b = rd_b == 2 * kBBytes ? 0 : rd_b + kBBytes;
 #pragma unroll
-    for (int kk = 0; kk < kKSteps; ++kk) { a_rd[kk] ^= kABytes; b_rd[kk] ^= kBBytes; }
-    // K step 1 of slab s, under it the reads of step 0 of slab s+1 and the loads of slab s+2
-    step(1, 0, 0, kLdT, full);
+    for (int kk = 0; kk < kKSteps; ++kk) { a_rd[kk] ^= kABytes; b_rd[kk] = b_rd0[kk] + rd_b; }
+    // K step 1 of slab s, under it the reads of step 0 of slab s+1 and the loads of A of slab s+2
+    step(1, 0, 0, kLA, full);
+    next_a();
   };
 
   const int nslab = (K + kTK - 1) / kTK;
-#pragma unroll
-  for (int l = 0; l < kL; ++l) issue_one(l, false);
-  next_slab();
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
   // past the last slab every lane is out of range: zeros go into the free buffer
 #pragma unroll
-  for (int l = 0; l < kLdT; ++l) issue_one(l, false);
+  for (int l = 0; l < kL; ++l) issue_one(l, false);
+  next_a();
+  next_b();
+#pragma unroll
+  for (int l = 0; l < kL; ++l) issue_one(l, false);
+  next_a();
+  next_b();
+  static_assert(kL == 16, "the loads of slab 1 may be on their way");
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
-  // slab s issues loads of slabs s+1 and s+2: no K-edge predicate while (s+3)*64 <= K
+  // slab s issues loads of slab s+2: no K-edge predicate while (s+3)*64 <= K
   const int nfull = max(K / kTK - 2, 0);
   int s = 0;
   for (; s < nfull; ++s) slab(true);

@@ -20,6 +20,23 @@ def test_gemm_nt_matches_fp32_reference(m, n, k):
     torch.testing.assert_close(got, ref, rtol=1e-2, atol=1e-2 * ref.abs().max().item() * 0.05)
 
 
+@pytest.mark.parametrize("k", [8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 448, 832])
+def test_products_over_few_slabs_of_the_contraction(k):
+    """One to thirteen slabs of 64, whole and cut short: every position of the rings of slab buffers at the start
+    and the end of a contraction, over a tile grid with ragged edges.  fp32 sums of k products of bf16 values,
+    rounded once: 2^-8 of a value, and of the sum's size 2^-8 again for values near zero."""
+    from speculators_amd.gemm import gemm_nt, gemm_tn, matmul_nn, matmul_nt
+
+    g = torch.Generator().manual_seed(k)
+    m, n = 520, 264
+    a, b = (torch.randn(r, k, generator=g).bfloat16().cuda() for r in (m, n))
+    ref = a.float() @ b.float().t()
+    bound = 2 ** -8 * (ref.abs() + k ** 0.5)
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    for out in (gemm_nt(a, b), matmul_nt(a, b), matmul_nn(a, bt), gemm_tn(at, bt)):
+        assert ((out.float() - ref).abs() <= bound).all()
+
+
 def test_gemm_strided_rows():
     from speculators_amd.gemm import gemm_nt
 
