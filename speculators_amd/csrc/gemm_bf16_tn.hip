@@ -17,13 +17,18 @@
 // piece position p ^ h(t), h(t) = t % 4 + 4 (t / 8 % 2): the 8 rows that one half of the lanes of a
 // read touches then cover all 64 banks once.
 //
-// From there on it is the NT kernel: 256 x 256 tile, 4 waves x 128 x 128 (one per SIMD), two
-// slab buffers, 8 x 8 accumulators of 16 x 16 per wave pinned to the accumulation registers, the LDS
-// reads of K step kk+1 and the global loads of the next slab issued one at a time between the MFMAs
+// From there on it is the NT kernel: 256 x 256 tile, 4 waves x 128 x 128 (one per SIMD), two slab
+// buffers of A and three of B, 8 x 8 accumulators of 16 x 16 per wave pinned to the accumulation registers, the
+// LDS reads of K step kk+1 and the global loads of slab s+2 issued one at a time between the MFMAs
 // of step kk, one barrier per slab, accumulators kept transposed (lane = row of C).  The slab loop is
-// written out for two slabs, so that the buffer a read goes to is a constant: a fragment read is an
-// address register per fragment plus an immediate, with no vector arithmetic between the MFMAs
+// written out for two slabs, so that the buffer of A a read goes to is a constant; B's addresses step on by a
+// buffer once a slab: a fragment read is an address register per fragment plus an immediate, and of vector
+// arithmetic between the MFMAs there are eight additions a slab and one per global load
 // (with 16-cycle MFMAs the kernel is bound by what a wave can issue, and every instruction counts).
+// The third buffer lets the loads follow each other evenly, one per eight MFMAs; with two all 16 of a slab came
+// behind the barrier, one per four, and each takes the wave's issue for longer than an MFMA takes the
+// matrix pipe.  Before / now, us: 28672 rows -> 4096 x 28672 4768 / 4517 (1491 TFLOP/s), -> 4096 x 14336 2633 / 2457,
+// -> 6144 x 8192 2026 / 1936; 98280 -> 6144 x 2048 2029 / 1896; 32000 -> 12288 x 2048 1356 / 1247; 1536 -> 16384 x 2048 92.5 / 90.7.
 
 #include "gemm_tile_api.h"
 #include "spx_common.h"
@@ -38,13 +43,13 @@ constexpr int kTM = 256, kTN = 256, kTK = 64;
 constexpr int kWM = 2, kWN = 2;
 constexpr int kMI = kTM / kWM / 16, kNI = kTN / kWN / 16;  // 8 x 8 accumulators of 16 x 16 per wave
 constexpr int kKSteps = kTK / 32;                          // MFMA K steps per slab
-#define SPX_GEMM_TN_READ_EVERY 2  // MFMAs per LDS fragment (two transposing reads) in the K step before the barrier
-#define SPX_GEMM_TN_READ_EVERY_B 4  // the same in the K step after it, which also issues the global loads
+#define SPX_GEMM_TN_READ_EVERY 2  // MFMAs per LDS fragment (two transposing reads), behind the odd ones
+#define SPX_GEMM_TN_LOAD_EVERY 8  // MFMAs per global -> LDS load, behind the first of them
 constexpr int kRowBytes = kTM * 2;                          // 512: one t-row of a slab
 constexpr int kABytes = kTK * kRowBytes;                    // one slab of A: 32 KB
 constexpr int kBBytes = kABytes;
 constexpr int kBBase = 2 * kABytes;
-constexpr int kSmem = 2 * (kABytes + kBBytes);              // 128 KB
+constexpr int kSmem = 2 * kABytes + 3 * kBBytes;            // 160 KB: all there is
 constexpr int kLA = kTK / 2 / kNW;                          // wave-loads (2 rows each) of A per wave per slab
 constexpr int kLB = kLA;
 constexpr int kL = kLA + kLB;
@@ -186,8 +191,8 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
   const uint32_t lds_a = lds0 + wave * kLA * 1024;
   const uint32_t lds_b = lds0 + kBBase + wave * kLB * 1024;
 
-  uint32_t bufoff = 0;  // slab buffer the next loads go to
-  int ld_t0 = 0;        // first row of the slab being loaded
+  uint32_t buf_a = 0, buf_b = 0;  // slab buffers the next loads go to
+  int ld_t0 = 0;                  // first row of the slab being loaded
   const int a_row = (int)(lda * 2), b_row = (int)(ldb * 2);
   // load l (A loads first, then B) of the slab at ld_t0
   auto issue_one = [&](int l) __attribute__((always_inline)) {
@@ -195,10 +200,11 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
     const int j = isa ? l : l - kLA;
     const uint32_t voff = (uint32_t)(isa ? aoff[j] : boff[j]) + (uint32_t)ld_t0 * (uint32_t)(isa ? a_row : b_row);
     // (a lane that is out of range stays so: kOob plus the row offset lies past any resource size)
-    load_to_lds16<0>(isa ? ares : bres, (isa ? lds_a : lds_b) + bufoff + j * 1024, (int)voff, 0);
+    load_to_lds16<0>(isa ? ares : bres, (isa ? lds_a + buf_a : lds_b + buf_b) + j * 1024, (int)voff, 0);
   };
   auto next_slab = [&]() __attribute__((always_inline)) {
-    bufoff ^= kABytes;
+    buf_a ^= kABytes;
+    buf_b = buf_b == 2 * kBBytes ? 0 : buf_b + kBBytes;
     ld_t0 += kTK;
     if (MULTI && ld_t0 >= T && seg < n_seg) {
       // this segment's rows are all requested: go on with the next segment that has rows (the
@@ -221,7 +227,8 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
   // read side (see the head of the file)
   const int trow = 8 * q + (r16 >> 2);
   const int lane_off = trow * kRowBytes + (((r16 >> 2) | ((q & 1) << 2)) * 32) + 8 * (r16 & 3);
-  uint32_t a_rd[kMI], b_rd[kNI];  // per fragment: LDS address in slab buffer 0
+  uint32_t a_rd[kMI], b_rd[kNI];  // per fragment: LDS address, of A in slab buffer 0, of B in the one that is read
+  uint32_t rd_b = 0;              // slab buffer of B that is read
 #pragma unroll
   for (int f = 0; f < kMI; ++f) {
     a_rd[f] = lds0 + (lane_off ^ ((wm / 16 + f) * 32));
@@ -232,10 +239,10 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
   }
 
   i16x4 fa[2][kMI][2], fb[2][kNI][2];
-  // operand fragment f (A fragments first, then B) of K step kk of slab buffer buf into register
+  // operand fragment f (A fragments first, then B) of K step kk of A's slab buffer buf and B's current one into register
   // set `set`; buf and kk are constants where this is called, so they end up in the offset field
   auto read_one = [&](int set, int buf, int kk, int f) __attribute__((always_inline)) {
-    const uint32_t o = buf * kABytes + kk * 32 * kRowBytes;
+    const uint32_t o = (f < kMI ? buf * kABytes : 0) + kk * 32 * kRowBytes;
     if (f < kMI) {
       fa[set][f][0] = lds_read_tr16_at(a_rd[f] + o);
       fa[set][f][1] = lds_read_tr16_at(a_rd[f] + o + 4 * kRowBytes);
@@ -249,8 +256,9 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
     return __builtin_bit_cast(bf16x8, v);
   };
   // One K step: the kNI x kMI MFMAs on register set `set`; between them, one at a time, the LDS
-  // reads that fill the other set with K step rk and the global loads [l0, l0 + nl).
-  auto step = [&](int set, int rbuf, int rk, int l0, int nl, int every) __attribute__((always_inline)) {
+  // reads that fill the other set with K step rk, the global loads [l0, l0 + nl) and (turn != 0) the
+  // steps of B's read addresses to the next slab buffer.
+  auto step = [&](int set, int rbuf, int rk, int l0, int nl, uint32_t turn) __attribute__((always_inline)) {
     constexpr int kN = kNI * kMI, kF = kMI + kNI;
     int reads = 0, loads = 0;
 #pragma unroll
@@ -260,43 +268,51 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
         mfma16(acc[j][i], frag(fb[set][j]), frag(fa[set][i]));
         const int idx = j * kMI + i;
         __builtin_amdgcn_sched_barrier(0);
-        if (reads < kF && idx % every == every - 1) {
+        if (reads < kF && idx % SPX_GEMM_TN_READ_EVERY == SPX_GEMM_TN_READ_EVERY - 1) {
           read_one(set ^ 1, rbuf, rk, reads++);
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (nl > 0 && (nl >= kN || idx % (kN / nl) == kN / nl - 1) && loads < nl) {
+        if (loads < nl && idx % SPX_GEMM_TN_LOAD_EVERY == 0) {
           issue_one(l0 + loads++);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (set == 1 && idx % 2 == 0 && idx / 2 < kNI) {
+          b_rd[idx / 2] += turn;
           __builtin_amdgcn_sched_barrier(0);
         }
       }
   };
 
-  // the loads of a slab are issued in the step after the barrier that frees its buffer, one per four
-  // MFMAs; the step after that gives them time to land
   static_assert(kKSteps == 2, "a slab is two K steps: one before, one after the barrier");
-  constexpr int kLdT = kL;
-  // buf: the buffer slab s lies in, a constant in each of the two copies of the loop body
+  // one slab: on entry set 0 holds (or is receiving) its K step 0 and the loads of slab s+1 are issued.
+  // buf: the buffer of A slab s lies in, a constant in each of the two copies of the loop body
   auto slab = [&](int buf) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    step(0, buf, 1, 0, 0, SPX_GEMM_TN_READ_EVERY);
-    next_slab();
-    // every read of this slab's buffer has returned once set 1 is complete; then the barrier says:
-    // slab s+1 has landed for everybody, this buffer is free
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // K step 0 of slab s, under it the reads of step 1 and the loads of B of slab s+2 into the third buffer
+    step(0, buf, 1, kLA, kLB, 0);
+    // every read of this slab's buffers has returned once set 1 is complete; then the barrier says:
+    // slab s+1 has landed for everybody, these buffers are free
+    static_assert(kLB == 8, "the loads of B of slab s+2 may be on their way");
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    // K step 1 of slab s, under it the reads of step 0 of slab s+1 and the loads of slab s+2
-    step(1, buf ^ 1, 0, 0, kLdT, SPX_GEMM_TN_READ_EVERY_B);
+    const uint32_t turn = rd_b == 2 * kBBytes ? 0u - 2 * kBBytes : kBBytes;
+    rd_b += turn;
+    // K step 1 of slab s, under it the reads of step 0 of slab s+1 and the loads of A of slab s+2
+    step(1, buf ^ 1, 0, 0, kLA, turn);
+    next_slab();
   };
 
   const int nslab = MULTI ? total_slabs : (T + kTK - 1) / kTK;
+  // (past the last slab every row is out of range: zeros go into the free buffer)
 #pragma unroll
   for (int l = 0; l < kL; ++l) issue_one(l);
   next_slab();
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  // (past the last slab every row is out of range: zeros go into the free buffer)
 #pragma unroll
-  for (int l = 0; l < kLdT; ++l) issue_one(l);
+  for (int l = 0; l < kL; ++l) issue_one(l);
+  next_slab();
+  static_assert(kL == 16, "the loads of slab 1 may be on their way");
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, 0, f);
   int s = 0;
