@@ -1,7 +1,7 @@
 // bf16 GEMM kernels for gfx950 on smaller tiles than those of gemm_bf16.hip (NT, NN and TN forms, plain, cut along
 // the contraction, grouped).  Instantiated, chosen and launched by gemm_tile.hip.
 //
-// Direct global -> LDS loads, STAGES slabs of 64 contraction indices deep, v_mfma_f32_16x16x32_bf16, operand
+// Direct global -> LDS loads, STAGES slabs of 64 contraction indices deep (ring_b), v_mfma_f32_16x16x32_bf16, operand
 // fragments double buffered in registers, the LDS reads of the next K step and the loads of the next free slab issued
 // between the products, one barrier per slab.  What bounds them is the way into LDS: with one tile on every compute unit
 // and K to 16384 the tiles of 64 x 128, 128 x 128 and 256 x 128 all load at 61 - 79 GB/s per compute unit (16 - 20 TB/s over
@@ -16,6 +16,8 @@
 // The weight gradients of 512 experts (2.1 GB from 80 rows each, operands in the memory-side cache, back to back) leave at
 // 3.2 TB/s as 64-byte pieces, 3.3 in whole lines, 3.6 past the caches and 4.6 with both.
 #pragma once
+
+#include <type_traits>
 
 #include "gemm_tile_api.h"
 #include "spx_common.h"
@@ -51,6 +53,16 @@ __device__ __forceinline__ void store_line(void* p, u32x4 v) {
   if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
   else *reinterpret_cast<u32x4*>(p) = v;
 }
+
+// Slab buffers of B where A has `stages`.  With two, B has a third, a free one at any time: its loads run under the first K
+// step of a slab, A's under the second, instead of all under the second.  Two of each / so, us: 3001 x 28672 -> 4096, NN 565
+// / 521, 8192 x 4096 -> 14336, NN 702 / 684, 1777 rows -> 2048 x 10240, TN 82.5 / 78.4, 64 groups of 1024 rows x 2048 -> 1536 403 /
+// 388, x 1536 -> 2048, NN 425 / 400.  (With three or four of each, B's loads half a slab later so that they follow each other
+// evenly: 0 - 5 % longer.)
+__host__ __device__ constexpr int ring_b(int stages) { return stages == 2 ? 3 : stages; }
+
+template <int N>
+using at = std::integral_constant<int, N>;
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -233,7 +245,11 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   constexpr int kWaves = WM * WN, kMI = TM / WM / 16, kNI = TN / WN / 16;
   using OA = Operand<TM, kWaves, AT>;
   using OB = Operand<TN, kWaves, BT>;
-  constexpr int kStage = OA::kBytes + OB::kBytes;
+  // slab buffers: A and B in turn, or where B has one more, all of A, then all of B
+  constexpr int kRingB = ring_b(STAGES);
+  constexpr bool kMoreB = kRingB > STAGES;
+  constexpr int kStage = kMoreB ? OA::kBytes : OA::kBytes + OB::kBytes;
+  constexpr int kBBase = kMoreB ? STAGES * kStage : OA::kBytes;
   constexpr int kL = OA::kLoads + OB::kLoads;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -310,7 +326,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   if constexpr (PICK == 2) ob.init_picked_slow(B + n0, p.ldb, p.N - n0, wave, lane, p.src_rows);
   else ob.init(BT ? B + n0 : B + (int64_t)n0 * p.ldb, p.ldb, p.N - n0, K, wave, lane);
   const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
-  const uint32_t a_rd = OA::read_base(lds0, wm, lane), b_rd = OB::read_base(lds0 + OA::kBytes, wn, lane);
+  const uint32_t a_rd = OA::read_base(lds0, wm, lane), b_rd = OB::read_base(lds0 + kBBase, wn, lane);
 
   f32x4 acc[kNI][kMI];
 #pragma unroll
@@ -320,7 +336,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
 
   const int nslab = (K + kTK - 1) / kTK;
   int ld_k = 0;  // contraction index of the slab being loaded
-  uint32_t ld_at = lds0;
+  uint32_t ld_at = lds0, ld_at_b = lds0 + kBBase;
   constexpr int kPick = AT ? PICK : 0;
   int picked[kPick == 1 ? OA::kLoads : OB::kLoads];  // rows of the slab that is loaded next
   auto pick = [&](int k0) __attribute__((always_inline)) {
@@ -332,20 +348,22 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
       if constexpr (kPick == 1) oa.load_picked(l, ld_at, picked, wave);
       else oa.load(l, ld_at, ld_k, K, wave);
     } else {
-      if constexpr (kPick == 2) ob.load_picked(l - OA::kLoads, ld_at + OA::kBytes, picked, wave);
-      else ob.load(l - OA::kLoads, ld_at + OA::kBytes, ld_k, K, wave);
+      const uint32_t to = kMoreB ? ld_at_b : ld_at + kBBase;
+      if constexpr (kPick == 2) ob.load_picked(l - OA::kLoads, to, picked, wave);
+      else ob.load(l - OA::kLoads, to, ld_k, K, wave);
     }
   };
   auto next_load = [&]() __attribute__((always_inline)) {
     ld_k += kTK;
     ld_at = ld_at + kStage == lds0 + STAGES * kStage ? lds0 : ld_at + kStage;
+    if (kMoreB) ld_at_b = ld_at_b + OB::kBytes == lds0 + kBBase + kRingB * OB::kBytes ? lds0 + kBBase : ld_at_b + OB::kBytes;
   };
   constexpr int kSets = STAGES == 1 ? 1 : 2;
   bf16x8 fa[kSets][kMI], fb[kSets][kNI];
-  uint32_t rd = 0;  // slab buffer the reads go to
+  uint32_t rd = 0, rd_b = 0;  // slab buffer the reads go to, and B's where it has more
   auto read_one = [&](int set, int kk, int f) __attribute__((always_inline)) {
     if (f < kMI) fa[set][f] = OA::read(a_rd, rd, wm, f, kk, lane);
-    else fb[set][f - kMI] = OB::read(b_rd, rd, wn, f - kMI, kk, lane);
+    else fb[set][f - kMI] = OB::read(b_rd, kMoreB ? rd_b : rd, wn, f - kMI, kk, lane);
   };
   // Grouped NT and NN: a wave whose rows are all past its group's loads and waits with the others, but multiplies nothing
   // (nor reads its operands, where there are several slab buffers): a group of 80 rows on average is half a tile.  4096 tokens, top 10 of 512 experts of uneven popularity, gate/up 470
@@ -354,17 +372,16 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
   constexpr bool kSkip = !AT && STREAM;
   const bool rows_here = !kSkip || __builtin_amdgcn_readfirstlane(m0 + wm < M);
   // One K step of 32: the products on register set `set`; between them the LDS reads that fill the other set with K
-  // step rk and (loads) the wave-loads of a whole slab
-  auto step = [&](int set, int rk, bool loads) __attribute__((always_inline)) {
+  // step rk and the wave-loads [first, last) of a slab
+  auto step = [&](int set, int rk, auto first, auto last) __attribute__((always_inline)) {
+    constexpr int kFirst = decltype(first)::value, kCount = decltype(last)::value - kFirst;
     if (kSkip && !rows_here) {
-      if (loads) {
 #pragma unroll
-        for (int l = 0; l < kL; ++l) issue_one(l);
-      }
+      for (int l = 0; l < kCount; ++l) issue_one(kFirst + l);
       return;
     }
     constexpr int kN = kNI * kMI, kF = kMI + kNI;
-    int reads = 0, issued = 0;
+    int reads = 0;
 #pragma unroll
     for (int j = 0; j < kNI; ++j)
 #pragma unroll
@@ -374,8 +391,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
         __builtin_amdgcn_sched_barrier(0);
         // reads in the first three quarters of the step, loads evenly
         while (reads < kF && reads * kN * 3 < (idx + 1) * kF * 4) { read_one(set ^ 1, rk, reads++); }
-        if (loads)
-          while (issued < kL && issued * kN < (idx + 1) * kL) issue_one(issued++);
+#pragma unroll
+        for (int l = 0; l < kCount; ++l)
+          if (l * kN / kCount == idx) issue_one(kFirst + l);
         __builtin_amdgcn_sched_barrier(0);
       }
   };
@@ -421,7 +439,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
       products();
     }
   } else {
-    // STAGES slab buffers (past the last slab the loads bring zeros)
+    // The loads of slab s + STAGES are issued under the second K step of slab s, B's under the first where it has a buffer
+    // more.  Past the last slab they bring zeros
 #pragma unroll
     for (int s = 0; s < STAGES; ++s) {
 #pragma unroll
@@ -435,14 +454,15 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
     for (int f = 0; f < kMI + kNI; ++f) read_one(0, 0, f);
     for (int s = 0; s < nslab; ++s) {
       __builtin_amdgcn_sched_barrier(0);
-      step(0, 1, false);
-      // every read of slab s has returned; after the barrier for every wave (its buffer is free) and slab s + 1 has
+      step(0, 1, at<OA::kLoads>{}, at<kMoreB ? kL : OA::kLoads>{});
+      // every read of slab s has returned; after the barrier for every wave (its buffers are free) and slab s + 1 has
       // landed for everybody
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kL) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kL + (kMoreB ? OB::kLoads : 0)) : "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       rd = rd + kStage == STAGES * kStage ? 0 : rd + kStage;
-      step(1, 0, true);
+      if (kMoreB) rd_b = rd_b + OB::kBytes == kRingB * OB::kBytes ? 0 : rd_b + OB::kBytes;
+      step(1, 0, at<0>{}, at<kMoreB ? OA::kLoads : kL>{});
       next_load();
     }
   }

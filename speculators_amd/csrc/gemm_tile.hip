@@ -62,7 +62,8 @@ constexpr int kPickRows = 256;  // rows a group on average up to which the group
 template <int TM, int TN, int WM, int WN, int STAGES, int MINB, bool AT, bool BT, int OUT, bool STREAM, bool GRADE = false,
           int PICK = 0>
 static int launch(const char* fname, Params p, int groups_y, hipStream_t st) {
-  constexpr int kSmem = (TM + TN) * kTK * 2 * STAGES;
+  constexpr int kSmem = (TM * STAGES + TN * ring_b(STAGES)) * kTK * 2;
+  static_assert(kSmem * (4 * MINB / (WM * WN)) <= 160 * 1024, "LDS for the workgroups that a compute unit shall hold");
   static std::atomic<uint64_t> lds_set;
   auto* const kernel = &gemm_tile_kernel<TM, TN, WM, WN, STAGES, MINB, AT, BT, OUT, STREAM, GRADE, PICK>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmem, lds_set, fname)) return rc;
