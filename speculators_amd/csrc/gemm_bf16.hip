@@ -36,42 +36,10 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_tile_api.h"
-#include "spx_common.h"
+#include "gemm_nt.h"
 #include "../../include/spx.h"
 
 namespace spx {
-
-#define SPX_GEMM_WM 2
-#define SPX_GEMM_WN 2
-#define SPX_GEMM_MINW 1
-#define SPX_GEMM_READ_EVERY 2  // MFMAs per LDS fragment read
-#define SPX_GEMM_LOAD_EVERY 8  // MFMAs per global -> LDS load ...
-#define SPX_GEMM_LOAD_AT 2     // ... of which the load follows this one (the reads follow the odd ones)
-constexpr int kWM = SPX_GEMM_WM, kWN = SPX_GEMM_WN;  // waves along M / N of the tile
-constexpr int kNW = kWM * kWN;
-constexpr int kGemmThreads = 64 * kNW;
-constexpr int kTM = 256, kTN = 256, kTK = 64;
-constexpr int kMI = kTM / kWM / 16, kNI = kTN / kWN / 16;  // 16x16 accumulators per wave
-constexpr int kKSteps = kTK / 32;                          // MFMA K steps per slab
-constexpr int kRowBytes = kTK * 2;                          // 128
-constexpr int kABytes = kTM * kRowBytes;                    // one slab of A: 32 KB
-constexpr int kBBytes = kTN * kRowBytes;
-constexpr int kBBase = 2 * kABytes;
-constexpr int kGemmSmem = 2 * kABytes + 3 * kBBytes;  // 160 KB: all there is
-constexpr int kLA = kTM / 8 / kNW;                  // wave-loads of A per wave per slab
-constexpr int kLB = kTN / 8 / kNW;
-constexpr int kL = kLA + kLB;
-constexpr int kOob = 0x7ffffff0;
-static_assert(kABytes == 32768 && kBBytes == 32768, "the buffer toggle flips bit 15");
-static_assert(kLA % 4 == 0 && kLB % 4 == 0, "loads are grouped in fours (immediate offsets)");
-
-__device__ __forceinline__ bf16x8 as_frag(u32x4 v) {
-  union { u32x4 u; bf16x8 b; } c;
-  c.u = v;
-  return c.b;
-}
-
 
 // kImm: consecutive loads of a group of four share one M0 value and differ in the
 // instruction's immediate offset (which moves the LDS and the global address alike, so
@@ -101,71 +69,6 @@ __device__ __forceinline__ int choose_k_parts(int n_tiles, int max_parts, int cu
 // float, sums as float, columns as int32); gemm_row_stats_reduce_kernel folds the tiles_n entries
 // of a row into log-sum-exp and arg-max.  C may then be null: the product itself is not stored
 // (a cross-entropy against arg-max targets needs nothing else of the target logits).
-// The tiles of the last, partly filled round of a product (n_tiles % cus of them, when they are at most
-// half a round): each is cut along the contraction into as many parts as fill the idle compute units
-// (at most max_parts, every part at least 16 slabs), so that the round takes a part's time instead of a
-// tile's.  384 tiles on 256 compute units: 256 whole tiles, then 128 tiles x 2 halves -- 1.5 rounds of
-// work in 1.5 rounds of time instead of 2.  first = index of the first tile that is cut (n_tiles: none).
-__host__ __device__ __forceinline__ void tail_plan(int n_tiles, int cus, int nslab, int max_parts, int& first,
-                                                   int& parts) {
-  first = n_tiles;
-  parts = 1;
-  if (n_tiles <= 0 || cus <= 0) return;
-  const int rem = n_tiles % cus;
-  if (rem == 0 || rem * 2 > cus) return;
-  int tp = cus / rem;
-  if (tp > max_parts) tp = max_parts;
-  while (tp > 1 && nslab / tp < 16) --tp;
-  if (tp > 1) { first = n_tiles - rem; parts = tp; }
-}
-
-// The same for a product whose rows are counted on the device, and for any last round: as many parts (at most max_parts, each
-// at least 16 slabs, tiles x parts at most `room` partial tiles) as make it shortest.  The times are those of the 256 x 256 tile,
-// as gemm_tile.hip has them, 16 us for a part's start and its 256 KB of partial results, and the pass behind it
-// (reduce_us there); one more part has to promise 3 %.  In whole numbers, nanoseconds times compute units: the product, the pass
-// that adds its parts and the host each work the plan out, and have to find the same one however they are compiled.
-// 400 tiles: 256 whole ones, then 144 in 5 parts, 3 / 5 of a round in the
-// place of one.  x 32000, us, all tiles cut in up to 4 parts (where there are at most 512) / so: -> 4096, 6300 live of 9003 rows
-// 1455 / 1300, 4500 of them 1416 / 898, 4200 of 6000 1042 / 867; -> 8192, 2150 of 3072 1020 / 865; -> 2048, 1260 of 1800
-// 173 / 154, 900 of them 152 / 116, 1800 of them 202 / 208; worst 1800 of 3600 200 / 209.
-__host__ __device__ __forceinline__ void live_tail_plan(int n_tiles, int cus, int nslab, int max_parts, int room, int& first,
-                                                        int& parts) {
-  first = n_tiles;
-  parts = 1;
-  const int rem = n_tiles > 0 ? n_tiles % cus : 0;
-  if (rem == 0) return;
-  auto rounds = [&](int wgs, int slabs) __attribute__((always_inline)) {
-    const int last = wgs % cus;
-    return (int64_t)slabs * ((int64_t)(wgs / cus) * 1410 * cus + (last ? 1180 * cus + 230 * last : 0));
-  };
-  int64_t best = rounds(rem, nslab) + 6900 * cus;
-  for (int p = 2; p <= max_parts && nslab / p >= 16 && rem * p <= room; ++p) {
-    const int64_t t = rounds(rem * p, (nslab + p - 1) / p) +
-                      (int64_t)cus * (16000 * ((rem * p + cus - 1) / cus) + 4100 + rem * p * 135 / 2);  // (67.5 ns a partial tile)
-    if (t * 100 < best * 97) { best = t; first = n_tiles - rem; parts = p; }
-  }
-}
-
-// tile index -> (tile row, tile column).  256 consecutive indices (what the chip runs at a time) are a block of
-// 16 x 16 tiles, so that a 256-row band of either operand is used by 16 of the tiles in flight, and the blocks walk
-// along the longer side of the tile grid; 32 consecutive indices (what one XCD runs: see the kernel) are 8 tiles
-// along the longer side x 4 along the shorter, 12 operand bands through that XCD's L2.  In detail: panels of 16
-// along the shorter side; inside a panel groups of 8 along the longer side; inside a group the longer side first.
-__device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int& tile_m, int& tile_n) {
-  constexpr int kPanel = 16, kGroup = 8;
-  const bool m_long = tiles_m >= tiles_n;
-  const int tl = m_long ? tiles_m : tiles_n, ts = m_long ? tiles_n : tiles_m;
-  const int panel = pid / (tl * kPanel);
-  const int ps = min(ts - panel * kPanel, kPanel);
-  const int p = pid - panel * tl * kPanel;
-  const int g = p / (kGroup * ps);
-  const int gsz = min(tl - g * kGroup, kGroup);
-  const int r = p - g * kGroup * ps;
-  const int l = g * kGroup + r % gsz, sh = panel * kPanel + r / gsz;
-  tile_m = m_long ? l : sh;
-  tile_n = m_long ? sh : l;
-}
-
 // kGrade: the rows are multiplied by their factors (RowGrade) on the way to their rounding.
 template <bool kImm, int kStats = 0, bool kGrade = false>
 __global__ __launch_bounds__(kGemmThreads, SPX_GEMM_MINW)
@@ -742,7 +645,6 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 3>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<false, 0, true>),
                               reinterpret_cast<const void*>(&gemm_bf16_nt_kernel<true, 0, true>)};
-  if (int rc = ensure_dynamic_lds(fns[which], kGemmSmem, lds_set[which], fname)) return rc;
   // grouped: every group may end in a partly filled tile row
   const int64_t tiles_m64 = (M + kTM - 1) / kTM + (tile_tab ? groups : 0);
   const int tiles_n = (int)((N + kTN - 1) / kTN);
@@ -760,25 +662,33 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
     n_grid = (int64_t)tiles_m * tiles_n + (int64_t)(tiles_m * tiles_n - tail_first) * (tail_parts - 1);
   }
   const dim3 grid((unsigned)n_grid), block(kGemmThreads);
+  // (row statistics, groups and products that are cut whole have a workgroup a tile)
+  if (!stat_ws && !tile_tab && (!part_ws || tail_mode) && walk_takes(false, c, ldb, ldc, N, K, n_grid)) {
+    const WalkArgs w = {reinterpret_cast<const uint16_t*>(a), lda, reinterpret_cast<const uint16_t*>(b), ldb,
+                        reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, part_ws, max_parts, tail_mode, cus, n_grid, grade};
+    if (int rc = walk(fname, false, w, st)) return rc;
+  } else {
+    if (int rc = ensure_dynamic_lds(fns[which], kGemmSmem, lds_set[which], fname)) return rc;
 #define SPX_GEMM_LAUNCH(IMM, ...)                                                                                \
   hipLaunchKernelGGL((gemm_bf16_nt_kernel<IMM, __VA_ARGS__>), grid, block, kGemmSmem, st,                        \
                      reinterpret_cast<const uint16_t*>(a), lda, reinterpret_cast<const uint16_t*>(b), ldb,       \
                      reinterpret_cast<uint16_t*>(c), ldc, (int)M, (int)N, (int)K, tiles_m, tiles_n, m_live,      \
                      tile_tab, group_off, b_group_stride, part_ws, max_parts, cus, stat_ws, tail_mode, grade)
-  switch (which) {
-    case 0: SPX_GEMM_LAUNCH(false, 0); break;
-    case 1: SPX_GEMM_LAUNCH(true, 0); break;
-    case 2: SPX_GEMM_LAUNCH(false, 1); break;
-    case 3: SPX_GEMM_LAUNCH(true, 1); break;
-    case 4: SPX_GEMM_LAUNCH(false, 2); break;
-    case 5: SPX_GEMM_LAUNCH(true, 2); break;
-    case 6: SPX_GEMM_LAUNCH(false, 3); break;
-    case 7: SPX_GEMM_LAUNCH(true, 3); break;
-    case 8: SPX_GEMM_LAUNCH(false, 0, true); break;
-    default: SPX_GEMM_LAUNCH(true, 0, true); break;
-  }
+    switch (which) {
+      case 0: SPX_GEMM_LAUNCH(false, 0); break;
+      case 1: SPX_GEMM_LAUNCH(true, 0); break;
+      case 2: SPX_GEMM_LAUNCH(false, 1); break;
+      case 3: SPX_GEMM_LAUNCH(true, 1); break;
+      case 4: SPX_GEMM_LAUNCH(false, 2); break;
+      case 5: SPX_GEMM_LAUNCH(true, 2); break;
+      case 6: SPX_GEMM_LAUNCH(false, 3); break;
+      case 7: SPX_GEMM_LAUNCH(true, 3); break;
+      case 8: SPX_GEMM_LAUNCH(false, 0, true); break;
+      default: SPX_GEMM_LAUNCH(true, 0, true); break;
+    }
 #undef SPX_GEMM_LAUNCH
-  if (int rc = check_launch(fname)) return rc;
+    if (int rc = check_launch(fname)) return rc;
+  }
   if (grade.row && !tail_mode) return 0;
   if (grade.row) {
     hipLaunchKernelGGL(gemm_tail_reduce_kernel<true>, dim3((unsigned)(std::min(tiles_m * tiles_n, cus - 1) * kTailSlices)),

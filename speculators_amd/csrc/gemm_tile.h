@@ -35,18 +35,6 @@ __device__ __forceinline__ i16x4 read_tr16(uint32_t addr) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(uintptr_t)addr);
 }
 
-// Two 16-byte pieces of one row, 64 bytes apart in memory, held by every lane (a wave: 16 rows x 4 lanes): lanes r and
-// r ^ 8 of a group of 16 exchange one piece each, after which the wave's first store (x) covers rows 0 .. 7 and its
-// second (y) rows 8 .. 15 in whole 128-byte lines.  lo: lane % 16 < 8; a lane's column is that of piece 0 if lo, else
-// of piece 1.
-__device__ __forceinline__ void line_pair(bool lo, u32x4 v0, u32x4 v1, u32x4& x, u32x4& y) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const uint32_t got = __builtin_amdgcn_update_dpp(0, lo ? v1[c] : v0[c], 0x128, 0xf, 0xf, true);  // row_ror:8
-    x[c] = lo ? v0[c] : got;
-    y[c] = lo ? got : v1[c];
-  }
-}
 // (a template argument: the compiler merges the two stores of a run-time choice into the cached one)
 template <bool STREAM>
 __device__ __forceinline__ void store_line(void* p, u32x4 v) {
@@ -393,7 +381,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void gemm_tile_kernel(Params p)
         while (reads < kF && reads * kN * 3 < (idx + 1) * kF * 4) { read_one(set ^ 1, rk, reads++); }
 #pragma unroll
         for (int l = 0; l < kCount; ++l)
-          if (l * kN / kCount == idx) issue_one(kFirst + l);
+          if (l * kN / (kCount > 0 ? kCount : 1) == idx) issue_one(kFirst + l);
         __builtin_amdgcn_sched_barrier(0);
       }
   };

@@ -545,6 +545,11 @@ static int auto_product(const char* fname, int form, const void* a, int64_t lda,
   p.part_ws = reinterpret_cast<float*>(workspace);
   p.m_live = m_live;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (form && ch.tile == tile::kFifth && walk_takes(true, c, ldb, ldc, N, K, tiles_m * tiles_n)) {
+    const WalkArgs w = {p.A, lda, p.B, ldb, reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, nullptr, 1, 0, tile::kCus,
+                        tiles_m * tiles_n, RowGrade{}};
+    return walk(fname, true, w, st);
+  }
   if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st))
     return rc;
   if (ch.parts == 1) return SPX_OK;

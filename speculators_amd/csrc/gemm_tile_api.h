@@ -25,6 +25,24 @@ int64_t nt_rows_graded_floats(int64_t M, int64_t N, int64_t K, int max_parts);
 // the parts of its last round of tiles for `live` rows
 int nt_rows_graded_parts(int64_t live, int64_t N, int64_t K, int64_t part_floats, int max_parts);
 
+// A product by workgroups that walk its tiles (gemm_bf16_walk.hip): a b^T or (slow) a b, n_grid = its tiles and the parts of
+// those that are cut; m_live, part_ws, max_parts, tail_mode, grade as in the 256 x 256 kernel of gemm_bf16.hip.  slow: no grade.
+struct WalkArgs {
+  const uint16_t* a;
+  int64_t lda;
+  const uint16_t* b;
+  int64_t ldb;
+  uint16_t* c;
+  int64_t ldc, M, N, K;
+  const int32_t* m_live;
+  float* part_ws;
+  int max_parts, tail_mode, cus;
+  int64_t n_grid;
+  RowGrade grade;
+};
+bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid);
+int walk(const char* fname, bool slow, const WalkArgs& w, hipStream_t st);
+
 namespace tile {
 
 int grouped_nt(const char* fname, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t b_group_stride,

@@ -123,6 +123,19 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Two 16-byte pieces of one row, 64 bytes apart in memory, held by every lane (a wave: 16 rows x 4 lanes): lanes r and
+// r ^ 8 of a group of 16 exchange one piece each, after which the wave's first store (x) covers rows 0 .. 7 and its
+// second (y) rows 8 .. 15 in whole 128-byte lines.  lo: lane % 16 < 8; a lane's column is that of piece 0 if lo, else
+// of piece 1.
+__device__ __forceinline__ void line_pair(bool lo, u32x4 v0, u32x4 v1, u32x4& x, u32x4& y) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t got = __builtin_amdgcn_update_dpp(0, lo ? v1[c] : v0[c], 0x128, 0xf, 0xf, true);  // row_ror:8
+    x[c] = lo ? v0[c] : got;
+    y[c] = lo ? got : v1[c];
+  }
+}
+
 // 64 lanes x 16 bytes, global -> LDS at M0 + IMM + 16 * lane; the global address is
 // base + voff + soff + IMM.  Lanes whose voff + IMM lies outside the resource write
 // zeros.  M0 is an input operand: the compiler writes it only when the value changes.
@@ -141,6 +154,20 @@ __device__ __forceinline__ void load_to_lds16(u32x4 rsrc, uint32_t lds_addr, int
     asm volatile("buffer_load_dwordx4 %1, %2, %3 offen offset:%4 lds"
                  :
                  : "{m0}"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM)
+                 : "memory");
+}
+
+// 16 bytes per lane to base + voff + IMM; lanes whose voff + IMM lies outside the resource store nothing.  One vector memory
+// operation whatever the lanes.  STREAM: past the caches.  (The scalar offset is in a register: without one, the instruction
+// behind a store of four words must not write these, and the compiler does not know that this is one.)
+template <int IMM, bool STREAM>
+__device__ __forceinline__ void buffer_store16(u32x4 rsrc, int voff, u32x4 v) {
+  const int zero = __builtin_amdgcn_readfirstlane(0);
+  if constexpr (STREAM)
+    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen offset:%4 nt" ::"v"(v), "v"(voff), "s"(rsrc), "s"(zero), "n"(IMM)
+                 : "memory");
+  else
+    asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen offset:%4" ::"v"(v), "v"(voff), "s"(rsrc), "s"(zero), "n"(IMM)
                  : "memory");
 }
 

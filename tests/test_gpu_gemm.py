@@ -37,6 +37,32 @@ def test_products_over_few_slabs_of_the_contraction(k):
         assert ((out.float() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("m,n,k,live", [
+    (256, 256, 192, None), (264, 256, 256, None),      # one tile of three slabs; a second of eight rows
+    (4352, 4096, 192, None),                           # 17 x 16 tiles: one round and a cut last one (3 slabs: too short to cut)
+    (4352, 4096, 2048, None), (8200, 4104, 320, None),  # its 16 last tiles in two parts; three rounds, ragged both ways
+    (4352, 4096, 2048, 4100), (4352, 4096, 2048, 1), (4352, 4096, 2048, 0)])  # rows counted on the device
+def test_products_of_workgroups_that_walk(m, n, k, live):
+    """The walking kernels against the fp32 product: tiles behind one another of a workgroup, the slabs of one in flight under the
+    last of the other, stores of whole tiles and of parts behind them, edges in rows and columns; the rest of the result is left
+    alone.  Bound: one rounding to bf16, and 2^-8 of the sum's size near zero."""
+    from speculators_amd.gemm import gemm_nt, matmul_nn
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    ref = a.float() @ b.float().t()
+    bound = 2 ** -8 * (ref.abs() + k ** 0.5)
+    rows = m if live is None else live
+    count = None if live is None else torch.tensor([live], dtype=torch.int32, device="cuda")
+    wide = torch.full((m + 1, n + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+    out = wide[:m, :n]
+    gemm_nt(a, b, out, count)
+    assert ((out[:rows].float() - ref[:rows]).abs() <= bound[:rows]).all()
+    assert (wide[rows:] == 7).all() and (wide[:, n:] == 7).all()
+    if live is None:
+        assert ((matmul_nn(a, b.t().contiguous()).float() - ref).abs() <= bound).all()
+
+
 def test_gemm_strided_rows():
     from speculators_amd.gemm import gemm_nt
 

@@ -156,3 +156,45 @@ def test_hand_issued_loads_are_not_read_before_their_wait(tmp_path):
                     assert not int(lo) <= int(reg[1:]) <= int(hi), f"{name}: {reg} inside {ins}"
         # the prologue and the two unrolled tiles issue eight loads each
         assert loads == 24 and waits >= 3, (name, loads, waits)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_named_accumulators_are_nobody_elses(tmp_path):
+    """The kernels that walk their tiles hold the accumulators in a0 .. a255 by name: no statement of the compiler's own touches
+    an accumulation register, none spills, and around every product lie the issue slots that it needs (as above; a fresh
+    product's result has no C operand)."""
+    text = _assembly("gemm_bf16_walk.hip", tmp_path)
+
+    def decimal(m):
+        return "a[" + ":".join(str(int(x, 0)) for x in m.group(1).split(":")) + "]" if ":" in m.group(1) else f"a{int(m.group(1), 0)}"
+
+    text = re.sub(r"\ba\[([\w:]+)\]", decimal, text)
+    kernels = 0
+    for m in re.finditer(r"^_ZN3spx21gemm_bf16_walk_kernel\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
+        kernels += 1
+        code, after = _flow(m.group(0).splitlines()[1:-1])
+        before = [[] for _ in code]
+        for n, nexts in enumerate(after):
+            for s in nexts:
+                before[s].append(n)
+        fresh = 0
+        for n, p in enumerate(code):
+            assert p.in_asm or not any(kind == "a" for kind, _ in p.all), p.text
+            assert not p.op.startswith("scratch_"), p.text
+            if not p.product:
+                continue
+            assert p.in_asm and (not p.c or p.c == p.d) and len(p.d) == 4
+            fresh += not p.c
+
+            def ahead(ins, between):
+                assert not (ins.writes & (p.a | p.b) and between < 2), (ins.text, between, p.text)
+
+            def behind(ins, between):
+                if ins.product and ins.d == p.d and not (ins.a | ins.b) & p.d:
+                    return True
+                assert not ins.all & p.d or between >= p.passes + 4, (p.text, between, ins.text)
+
+            _walk(before[n], before, code, 2, ahead)
+            _walk(after[n], after, code, 12, behind)
+        assert fresh == 64 and sum(p.product for p in code) == 256
+    assert kernels == 6
