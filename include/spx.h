@@ -883,6 +883,27 @@ int spx_gemm_bf16_tn_f32(const void* a, int64_t lda, const void* b, int64_t ldb,
                          void* c, int64_t ldc, int64_t M, int64_t N, int64_t T,
                          int accumulate, void* stream);
 
+/* One weight gradient c[M, N] = a[T, M]^T b[T, N] of a list; ldc in elements of c. */
+typedef struct spx_tn_product {
+  const void* a;
+  int64_t lda;
+  const void* b;
+  int64_t ldb;
+  void* c;
+  int64_t ldc, M, N, T;
+} spx_tn_product;
+
+/* 1 .. 8 weight gradients in one launch, bf16 or (out_f32) fp32: the 256 x 256 tiles of all of them are walked by one workgroup
+ * per compute unit, products of long contractions first, and those of the last round are cut along the contraction where that
+ * is shorter and `workspace` (16-byte aligned, may be NULL) holds their fp32 partial results; these are added in a fixed order.
+ * Rules of the two entry points above, but operands of any span; and T at least 129, lda and ldb at least 256, c 16-byte aligned
+ * with a leading dimension that is a multiple of 8 (spx_gemm_tn_list_us: microseconds it is predicted to take, -1 where it is
+ * not taken).  spx_gemm_tn_list_workspace_bytes: what the workspace has to hold to be used. */
+int64_t spx_gemm_tn_list_workspace_bytes(const spx_tn_product* products, int n, int out_f32);
+float spx_gemm_tn_list_us(const spx_tn_product* products, int n, int out_f32);
+int spx_gemm_bf16_tn_list(const spx_tn_product* products, int n, int out_f32, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
 /* Either of the two (out_f32) on the tiles its size asks for: results of few 256 x 256 tiles run on smaller ones, small
  * results over many rows with the contraction in parts (fp32 partials in `workspace`, added in a fixed order, with what c
  * holds where the product accumulates, one rounding).  workspace may be NULL (never cut); spx_gemm_tn_parts says into how
@@ -892,6 +913,8 @@ int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T);
  * waves, 2: 256 x 128, 3: 64 x 128, 4: 128 x 128 by four waves, two workgroups to a compute unit */
 int spx_gemm_tn_tile(int64_t M, int64_t N, int64_t T);
 int64_t spx_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t T);
+/* microseconds such a product is predicted to take */
+float spx_gemm_tn_us(int64_t M, int64_t N, int64_t T);
 int spx_gemm_bf16_tn_auto(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
                           int64_t N, int64_t T, int out_f32, int accumulate, void* workspace, int64_t workspace_bytes,
                           void* stream);

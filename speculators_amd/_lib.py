@@ -121,6 +121,10 @@ SIGNATURES["spx_gemm_bf16_rows_graded"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _
 SIGNATURES["spx_gemm_bf16_tn"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _P]
 SIGNATURES["spx_gemm_bf16_tn_auto"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P]
 SIGNATURES["spx_gemm_tn_parts"] = [_I64, _I64, _I64]
+SIGNATURES["spx_gemm_tn_us"] = [_I64, _I64, _I64]
+SIGNATURES["spx_gemm_bf16_tn_list"] = [_P, _I, _I, _P, _I64, _P]
+SIGNATURES["spx_gemm_tn_list_us"] = [_P, _I, _I]
+SIGNATURES["spx_gemm_tn_list_workspace_bytes"] = [_P, _I, _I]
 SIGNATURES["spx_gemm_tn_tile"] = [_I64, _I64, _I64]
 SIGNATURES["spx_gemm_tn_workspace_bytes"] = [_I64, _I64, _I64]
 SIGNATURES["spx_gemm_bf16_tn_f32"] = [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I, _P]
@@ -157,7 +161,7 @@ SIGNATURES["spx_gemm_graded_parts"] = [_I64, _I64, _I64, _I32, _I32, _I64, _I64]
 SIGNATURES["spx_gemm_bf16_auto_parts"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P]
 SIGNATURES["spx_gemm_bf16_auto"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P]
 SIGNATURES["spx_stage_upload"] = [_P, _I64, _P, _P, _I64, _I32, _P]
-RESTYPES = {"spx_gemm_auto_workspace_bytes": c_int64, "spx_gemm_graded_workspace_bytes": c_int64, "spx_gemm_tn_workspace_bytes": c_int64, "spx_gemm_auto_us": c_float, "spx_moe_sort_workspace_bytes": c_int64, "spx_loss_steps_partials": c_int64, "spx_gemm_grouped_workspace_bytes": c_int64, "spx_gemm_tail_workspace_bytes": c_int64, "spx_gemm_stats_workspace_bytes": c_int64, "spx_gemm_split_workspace_bytes": c_int64, "spx_ttt_attn_workspace_bytes": c_int64, "spx_ttt_attn_fwd_static_max_bytes": c_int64, "spx_dflash_attn_workspace_bytes": c_int64,
+RESTYPES = {"spx_gemm_auto_workspace_bytes": c_int64, "spx_gemm_graded_workspace_bytes": c_int64, "spx_gemm_tn_workspace_bytes": c_int64, "spx_gemm_auto_us": c_float, "spx_gemm_tn_us": c_float, "spx_gemm_tn_list_us": c_float, "spx_gemm_tn_list_workspace_bytes": c_int64, "spx_moe_sort_workspace_bytes": c_int64, "spx_loss_steps_partials": c_int64, "spx_gemm_grouped_workspace_bytes": c_int64, "spx_gemm_tail_workspace_bytes": c_int64, "spx_gemm_stats_workspace_bytes": c_int64, "spx_gemm_split_workspace_bytes": c_int64, "spx_ttt_attn_workspace_bytes": c_int64, "spx_ttt_attn_fwd_static_max_bytes": c_int64, "spx_dflash_attn_workspace_bytes": c_int64,
             "spx_rmsnorm_bwd_slots": c_int64}
 
 _lib = None

@@ -130,6 +130,7 @@ PyMethodDef g_methods[] = {
     SPX_HOST("normed_forward", spx_layer_normed_forward)
     SPX_HOST("normed_backward", spx_layer_normed_backward)
     SPX_HOST("product_tn", spx_layer_product_tn)
+    SPX_HOST("products_tn", spx_layer_products_tn)
     SPX_HOST("loss_step", spx_layer_loss_step)
     SPX_HOST("loss_terms", spx_layer_loss_terms)
     SPX_HOST("loss_steps_begin", spx_layer_loss_steps_begin)

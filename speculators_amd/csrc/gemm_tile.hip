@@ -647,6 +647,11 @@ extern "C" int32_t spx_gemm_tn_parts(int64_t M, int64_t N, int64_t T) {
   return tile::choose_tn(M, N, T, true).parts;
 }
 
+extern "C" float spx_gemm_tn_us(int64_t M, int64_t N, int64_t T) {
+  if (M <= 0 || N <= 0 || T <= 0) return 0.f;
+  return tile::choose_tn(M, N, T, true).us;
+}
+
 extern "C" int spx_gemm_tn_tile(int64_t M, int64_t N, int64_t T) {
   if (M <= 0 || N <= 0 || T <= 0) return 0;
   return tile::choose_tn(M, N, T, true).tile;

@@ -379,6 +379,47 @@ PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Weight gradients in one launch: (fp32, workspace or None, then for each a [T, M], b [T, N], out [M, N] or None)
+// -> the results
+PyObject* spx_layer_products_tn(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n >= 5 && n % 3 == 2 && n <= 26, "products_tn takes three arguments for each of 1 .. 8 products, and two");
+  Args x("products_tn", args, n, n);
+  const int64_t f32 = x.integer();
+  const Tensor ws = x.maybe();
+  const int count = (int)(n / 3);
+  Tensor a[8], b[8], out[8];
+  for (int i = 0; i < count; ++i) {
+    a[i] = x.tensor();
+    b[i] = x.tensor();
+    out[i] = x.maybe();
+    TORCH_CHECK_VALUE(a[i].dim() == 2 && b[i].dim() == 2 && a[i].size(0) == b[i].size(0) && a[i].stride(1) == 1 && b[i].stride(1) == 1 &&
+                          a[i].scalar_type() == at::kBFloat16 && b[i].scalar_type() == at::kBFloat16 && a[i].device() == a[0].device() &&
+                          b[i].device() == a[0].device(),
+                      "bf16 operands [T, M], [T, N] with contiguous rows, on one device");
+    TORCH_CHECK_VALUE(!out[i].defined() || (out[i].dim() == 2 && out[i].size(0) == a[i].size(1) && out[i].size(1) == b[i].size(1) &&
+                                            out[i].stride(1) == 1 && out[i].scalar_type() == (f32 ? at::kFloat : at::kBFloat16) &&
+                                            out[i].device() == a[0].device()),
+                      "out does not fit its product");
+  }
+  Unlocked released;
+  spx_tn_product list[8];
+  for (int i = 0; i < count; ++i) {
+    if (!out[i].defined())
+      out[i] = at::empty({a[i].size(1), b[i].size(1)}, a[i].options().dtype(f32 ? at::kFloat : at::kBFloat16).requires_grad(false));
+    list[i] = {in(a[i]), a[i].stride(0), in(b[i]), b[i].stride(0), out[i].mutable_data_ptr(), out[i].stride(0),
+               a[i].size(1), b[i].size(1), a[i].size(0)};
+  }
+  check(spx_gemm_bf16_tn_list(list, count, (int)f32, ws.defined() ? ws.mutable_data_ptr() : nullptr,
+                              ws.defined() ? (int64_t)ws.nbytes() : 0, stream_of(a[0])),
+        "spx_gemm_bf16_tn_list");
+  released.lock();
+  PyObject* const all = PyTuple_New(count);
+  for (int i = 0; i < count; ++i) PyTuple_SET_ITEM(all, i, THPVariable_Wrap(out[i]));
+  return all;
+  END_HANDLE_TH_ERRORS
+}
+
 // One TTT step's loss over bf16 logits in one read of the rows, with its masked mean: (op, logits, targets or None, known
 // lse_t, known argmax_t or None, mask, its kind, prev or None, its kind, acceptance counts or None (made and cleared here),
 // loss so far or None, step weight, term factor, scalars [8] or None: no mean) -> (total, row losses, argmax_draft,

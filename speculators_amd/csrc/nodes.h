@@ -17,6 +17,7 @@ PyObject* spx_layer_ttt_backward(PyObject*, PyObject* const* args, Py_ssize_t n)
 PyObject* spx_layer_normed_forward(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_normed_backward(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_product_tn(PyObject*, PyObject* const* args, Py_ssize_t n);
+PyObject* spx_layer_products_tn(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_step(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_terms(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_loss_steps_begin(PyObject*, PyObject* const* args, Py_ssize_t n);

@@ -66,6 +66,13 @@ def _check_param_dtype(p: torch.Tensor):
         "weights and run the forward under torch.autocast(dtype=torch.bfloat16)")
 
 
+def _check_params(params):
+    for p in params:
+        _check_param_dtype(p)
+        if not p.is_cuda:
+            raise _lib.SpxError("libspx_hip works on HIP device tensors only (got a CPU parameter)")
+
+
 _CAST_PARTS = 8  # matrices of one launch
 
 
@@ -149,20 +156,19 @@ def wgrad_product(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor | None) -
     return torch.addmm(acc, dy.t(), x, out_dtype=torch.float32, out=acc)
 
 
-class Staged:
-    """One compute weight of this forward.  ``w``: bf16 ``[rows, cols]`` (or 1-D for a norm gain);
-    ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward
-    is expected to run against it (the size of the input / output-gradient buffers)."""
+class _Uses:
+    """The uses of one compute weight in a forward and its backward: the inputs they ran on and the output gradients that came
+    back.  What the staging node holds -- not the ``Staged`` itself, whose token leads back to the node."""
 
-    __slots__ = ("w", "token", "rows_of", "uses", "_wt", "_xs", "_fill", "_dys", "_live", "_extras",
-                 "_marked", "_acc", "_task", "applied", "bf16_params")
+    __slots__ = ("shape", "device", "uses", "trainable", "bf16_params", "applied", "_xs", "_fill", "_dys", "_live", "_extras",
+                 "_marked", "_acc", "_task")
 
-    def __init__(self, w, rows_of, uses: int = 1, bf16_params: bool = False):
-        self.w = w
-        self.token = None  # fp32 stand-in of w's shape that carries the gradient edge (trainable only)
-        self.rows_of = rows_of
+    def __init__(self, uses: int, bf16_params: bool):
+        self.shape = self.device = None  # of the compute weight
         self.uses = uses
-        self._wt = None
+        self.trainable = False
+        self.bf16_params = bf16_params  # the parameters are bf16: a gradient written once may be bf16 itself
+        self.applied = 0   # products of this forward that add their gradient to _acc
         self._xs = None    # [uses * T, cols]: the inputs of the uses, one after the other
         self._fill = 0     # rows of _xs taken by products so far
         self._dys = None   # [uses * T, rows]: the output gradients, same row positions (backward only)
@@ -170,34 +176,17 @@ class Staged:
         self._extras = []  # (dy, x) of uses outside the buffers
         self._marked = False
         self._acc = None   # gradient buffer of uses that add their gradient themselves
-        self.applied = 0   # products of this forward whose gradient goes to that buffer
-        self.bf16_params = bf16_params  # the parameters are bf16: a gradient written once may be bf16 itself
         self._task = None     # the backward pass (autograd graph task) the recorded uses belong to
-
-    @property
-    def trainable(self) -> bool:
-        return self.token is not None
-
-    @property
-    def has_wt(self) -> bool:
-        return self._wt is not None
-
-    @property
-    def wt(self) -> torch.Tensor:
-        """``w.T`` contiguous (made on first use, kept with the staged weight)."""
-        if self._wt is None:
-            self._wt = transposed_copy(self.w.detach())
-        return self._wt
 
     # ---- forward side
     def x_slot(self, rows: int):
         """Where the input ``[rows, cols]`` of the next product against this weight should be
         written so that its weight gradient joins the one product over all uses; None when
         there is nothing to gain (frozen weight, no graph, a single use) or no room."""
-        if self.token is None or self.uses <= 1 or not torch.is_grad_enabled():
+        if not self.trainable or self.uses <= 1 or not torch.is_grad_enabled():
             return None
         if self._xs is None:
-            self._xs = torch.empty(self.uses * rows, self.w.shape[1], device=self.w.device,
+            self._xs = torch.empty(self.uses * rows, self.shape[1], device=self.device,
                                    dtype=torch.bfloat16)
         if self._fill + rows > self._xs.shape[0]:
             return None
@@ -233,7 +222,7 @@ class Staged:
             return None
         self._enter_pass()
         if self._dys is None:
-            self._dys = torch.empty(self._xs.shape[0], self.w.shape[0], device=self.w.device,
+            self._dys = torch.empty(self._xs.shape[0], self.shape[0], device=self.device,
                                     dtype=torch.bfloat16)
         return self._dys[r0:r0 + rows]
 
@@ -257,7 +246,7 @@ class Staged:
         if self._marked:
             return None
         self._marked = True
-        return _lib.zero(self.w.device).expand(self.w.shape)
+        return _lib.zero(self.device).expand(self.shape)
 
     def grad_buffer(self):
         """``(buffer, holds)``: the buffer of ``w``'s shape that uses which compute their weight
@@ -269,9 +258,26 @@ class Staged:
         holds = self._acc is not None
         if not holds:
             once = self.bf16_params and self.applied == 1
-            self._acc = torch.empty(self.w.shape, device=self.w.device,
+            self._acc = torch.empty(self.shape, device=self.device,
                                     dtype=torch.bfloat16 if once else torch.float32)
         return self._acc, holds
+
+    def sole(self):
+        """``(dy, x)`` where one product is all there is to the weight gradient (the records are dropped then), else None."""
+        if self._acc is not None or len(self._extras) > 1 or bool(self._extras) == bool(self._live):
+            return None
+        if self._extras:
+            pair = self._extras[0]
+        else:
+            live = sorted(self._live)
+            if any(a + n != b for (a, n), (b, _) in zip(live, live[1:], strict=False)):
+                return None
+            rows = slice(live[0][0], live[-1][0] + live[-1][1])
+            pair = self._dys[rows], self._xs[rows]
+        if not (_tn_ok(pair[0]) and _tn_ok(pair[1])):
+            return None
+        self._dys, self._live, self._extras, self._marked = None, [], [], False
+        return pair
 
     def finish(self, bf16_ok: bool = False):
         """The fp32 weight gradient of every recorded use (None if there is none): one product
@@ -308,19 +314,67 @@ class Staged:
         return acc
 
 
+class Staged:
+    """One compute weight of this forward.  ``w``: bf16 ``[rows, cols]`` (or 1-D for a norm gain);
+    ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward
+    is expected to run against it (the size of the input / output-gradient buffers)."""
+
+    __slots__ = ("w", "token", "rows_of", "_wt", "records", "x_slot", "take", "dy_slot", "defer", "mark", "grad_buffer")
+
+    def __init__(self, w, rows_of, uses: int = 1, bf16_params: bool = False):
+        self.w = w
+        self.token = None  # fp32 stand-in of w's shape that carries the gradient edge (trainable only)
+        self.rows_of = rows_of
+        self._wt = None
+        r = self.records = _Uses(uses, bf16_params)
+        self.x_slot, self.take = r.x_slot, r.take
+        self.dy_slot, self.defer, self.mark, self.grad_buffer = r.dy_slot, r.defer, r.mark, r.grad_buffer
+
+    def train(self, w, token):
+        """The compute weight and its token, as the staging node made them."""
+        self.w, self.token = w, token
+        r = self.records
+        r.shape, r.device, r.trainable = w.shape, w.device, True
+
+    @property
+    def trainable(self) -> bool:
+        return self.token is not None
+
+    @property
+    def uses(self) -> int:
+        return self.records.uses
+
+    @property
+    def applied(self) -> int:
+        return self.records.applied
+
+    @applied.setter
+    def applied(self, n: int):
+        self.records.applied = n
+
+    @property
+    def has_wt(self) -> bool:
+        return self._wt is not None
+
+    @property
+    def wt(self) -> torch.Tensor:
+        """``w.T`` contiguous (made on first use, kept with the staged weight)."""
+        if self._wt is None:
+            self._wt = transposed_copy(self.w.detach())
+        return self._wt
+
+
 class _Stage(torch.autograd.Function):
     """params -> (their bf16 row-wise concatenation, the fp32 token that carries its gradient);
-    backward: the weight-gradient product over all recorded uses (``Staged.finish``), split and
+    backward: the weight-gradient product over all recorded uses (``_Uses.finish``), split and
     cast to each parameter's dtype."""
 
     @staticmethod
-    def forward(ctx, staged: Staged, made: tuple, *params):
-        ctx.staged = staged
+    def forward(ctx, records: _Uses, *params):
+        ctx.records = records
         ctx.rows = [p.shape[0] for p in params]
         ctx.dtypes = [p.dtype for p in params]
-        if made:
-            w, = made
-        elif len(params) == 1 and params[0].dtype == torch.bfloat16:
+        if len(params) == 1 and params[0].dtype == torch.bfloat16:
             w = _as_it_lies(params[0])
         else:
             w = _cat_bf16(params)
@@ -331,23 +385,74 @@ class _Stage(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, _gw, g):
-        # g is the marker of ``Staged.defer`` (no memory behind it): the gradient is computed here,
+        # g is the marker of ``_Uses.defer`` (no memory behind it): the gradient is computed here,
         # now that every use has run its backward
-        acc = ctx.staged.finish(bf16_ok=all(dt == torch.bfloat16 for dt in ctx.dtypes))
+        acc = ctx.records.finish(bf16_ok=all(dt == torch.bfloat16 for dt in ctx.dtypes))
         if acc is not None:
             g = acc
         if g is None:
-            return (None,) * (2 + len(ctx.rows))
-        parts = g.split(ctx.rows, dim=0) if len(ctx.rows) > 1 else (g,)
-        grads = []
-        for i, (part, dt) in enumerate(zip(parts, ctx.dtypes, strict=True)):
-            if not ctx.needs_input_grad[2 + i]:
-                grads.append(None)
-            elif part.dtype == dt and len(parts) == 1:
-                grads.append(part)
+            return (None,) * (1 + len(ctx.rows))
+        return (None, *_param_grads(g, ctx.rows, ctx.dtypes, ctx.needs_input_grad[1:]))
+
+
+def _param_grads(g, rows, dtypes, needed):
+    """The gradients of the parameters that a compute weight with gradient ``g`` is made of."""
+    parts = g.split(rows, dim=0) if len(rows) > 1 else (g,)
+    # (a part of a merged buffer is copied where its dtype changes)
+    return [part.to(dt) if need else None for part, dt, need in zip(parts, dtypes, needed, strict=True)]
+
+
+class _StageAll(torch.autograd.Function):
+    """``_Stage`` of several compute weights whose uses end together (the weights of a layer): their weight gradients are one
+    launch where that is faster (``gemm.gemm_tn_all``)."""
+
+    @staticmethod
+    def forward(ctx, records, made, sizes, *params):
+        ctx.records, ctx.sizes = records, sizes
+        ctx.rows, ctx.dtypes = [p.shape[0] for p in params], [p.dtype for p in params]
+        ctx.set_materialize_grads(False)
+        out, at = [], 0
+        for i, n in enumerate(sizes):
+            group = params[at:at + n]
+            at += n
+            w = made.get(i)
+            if w is None:
+                w = _as_it_lies(group[0]) if n == 1 and group[0].dtype == torch.bfloat16 else _cat_bf16(group)
+            out += [w, _lib.zero(w.device).expand(w.shape)]
+        ctx.mark_non_differentiable(*out[::2])
+        return tuple(out)
+
+    @staticmethod
+    def backward(ctx, *gs):
+        from .gemm import gemm_tn_all
+
+        needed = ctx.needs_input_grad[3:]
+        groups, at = [], 0
+        for n in ctx.sizes:
+            groups.append(slice(at, at + n))
+            at += n
+        sums, together = [None] * len(groups), {torch.bfloat16: [], torch.float32: []}
+        for i, (uses, group) in enumerate(zip(ctx.records, groups, strict=True)):
+            g = gs[2 * i + 1]
+            if not any(needed[group]):
+                continue
+            bf16 = all(dt == torch.bfloat16 for dt in ctx.dtypes[group])
+            pair = uses.sole()
+            if pair is not None:
+                together[torch.bfloat16 if bf16 else torch.float32].append((i, pair))
             else:
-                grads.append(part.to(dt))  # a copy: the parts of a merged buffer become independent
-        return (None, None, *grads)
+                sums[i] = uses.finish(bf16_ok=bf16)
+                if sums[i] is None:
+                    sums[i] = g
+        for dtype, members in together.items():
+            if members:
+                for (i, _), acc in zip(members, gemm_tn_all([pair for _, pair in members], dtype), strict=True):
+                    sums[i] = acc
+        grads = []
+        for g, group in zip(sums, groups, strict=True):
+            grads += [None] * (group.stop - group.start) if g is None else _param_grads(
+                g, ctx.rows[group], ctx.dtypes[group], needed[group])
+        return (None, None, None, *grads)
 
 
 class _StageGains(torch.autograd.Function):
@@ -409,32 +514,37 @@ class WeightStager:
         self._fwd = {}
 
     def get_all(self, *groups):
-        """``get`` of every group of parameters (None: None), those that have to be cast in one launch."""
-        made = {}
+        """``get`` of every group of parameters (None: None): those that train are staged by one node, and those that have to be
+        cast are cast in one launch."""
         if torch.is_grad_enabled():
-            new = [i for i, g in enumerate(groups) if g is not None and tuple(id(p) for p in g) not in self._fwd]
-            if len(new) > 1 and _autocast_bf16(groups[new[0]][0].device.type):
-                made = dict(zip(new, _cast_together([groups[i] for i in new]) or (), strict=False))
-        return tuple(None if g is None else self._get(g, made.get(i)) for i, g in enumerate(groups))
+            new = {tuple(id(p) for p in g): g for g in groups if g is not None}
+            new = [g for key, g in new.items() if key not in self._fwd]
+            train = [g for g in new if any(p.requires_grad for p in g)]
+            if len(train) > 1:
+                self._stage_all(train, _cast_together(new) if _autocast_bf16(new[0][0].device.type) else None)
+        return tuple(None if g is None else self.get(*g) for g in groups)
+
+    def _stage_all(self, groups, made):
+        """``made``: their bf16 copies where they are there already."""
+        for g in groups:
+            _check_params(g)
+        staged = [Staged(None, [p.shape[0] for p in g], self._uses, all(p.dtype == torch.bfloat16 for p in g)) for g in groups]
+        out = _StageAll.apply([st.records for st in staged], dict(enumerate(made or ())), [len(g) for g in groups], *(p for g in groups for p in g))
+        for st, g, w, token in zip(staged, groups, out[::2], out[1::2], strict=True):
+            st.train(w, token)
+            self._fwd[tuple(id(p) for p in g)] = st
 
     def get(self, *params) -> Staged:
         """The staged row-wise concatenation of ``params`` for the running forward."""
-        return self._get(params)
-
-    def _get(self, params, made=None) -> Staged:
-        """``made``: their bf16 copy where it is there already."""
         key = tuple(id(p) for p in params)
         hit = self._fwd.get(key)
         if hit is not None:
             return hit
-        for p in params:
-            _check_param_dtype(p)
-            if not p.is_cuda:
-                raise _lib.SpxError("libspx_hip works on HIP device tensors only (got a CPU parameter)")
+        _check_params(params)
         rows_of = [p.shape[0] for p in params]
         if torch.is_grad_enabled() and any(p.requires_grad for p in params):
             st = Staged(None, rows_of, self._uses, all(p.dtype == torch.bfloat16 for p in params))
-            st.w, st.token = _Stage.apply(st, () if made is None else (made,), *params)
+            st.train(*_Stage.apply(st.records, *params))
         else:
             fkey = tuple((p.data_ptr(), p._version, p.dtype) for p in params)
             kept = self._frozen.get(key)

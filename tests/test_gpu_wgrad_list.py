@@ -1,0 +1,115 @@
+"""Weight gradients of several products in one launch (spx_gemm_bf16_tn_list), and the node that stages a layer's weights together."""
+
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+LISTS = {
+    "one tile of three slabs, the last of a row": [(129, 256, 256)],
+    "ragged results, contractions that end inside a slab": [(200, 264, 520), (1000, 1032, 256), (130, 256, 1000)],
+    "a last round in parts": [(4100, 512, 768)],
+    "whole rounds, then one in parts of unlike contractions": [(2112, 4096, 4096), (2049, 264, 2048), (2304, 520, 256)],
+    "a long tile first and a short last round": [(2665, 512, 512), (300, 4096, 4096), (200, 1032, 512)],
+    "eight": [(130 + 64 * i, 256 + 8 * i, 520) for i in range(8)]}
+
+
+def _operands(shapes, pad=0):
+    g = torch.Generator(device="cuda").manual_seed(len(shapes))
+    new = lambda t, n: torch.randn(t, n + pad, device="cuda", generator=g).bfloat16()[:, :n]  # noqa: E731
+    return [(new(t, m), new(t, n)) for t, m, n in shapes]
+
+
+@pytest.mark.parametrize("name", LISTS)
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_list_against_float64(name, fp32, pad):
+    """fp32 sums of t products, and one rounding to bf16; rows and columns beside a result are left alone."""
+    from speculators_amd.gemm import _tn_list
+
+    shapes = LISTS[name]
+    pairs = _operands(shapes, pad)
+    wide = [torch.full((m + 1, n + 8), 3.0, device="cuda", dtype=torch.float32 if fp32 else torch.bfloat16) for _, m, n in shapes]
+    outs = [w[:m, :n] for w, (_, m, n) in zip(wide, shapes)]
+    for _ in range(2):
+        _tn_list(pairs, fp32, outs)
+        for (a, b), out, w, (t, m, n) in zip(pairs, outs, wide, shapes):
+            want = a.double().t() @ b.double()
+            tol = (2e-6 * t ** 0.5 if fp32 else 2 ** -8) * want.abs().max().item() + 1e-4
+            assert (out.double() - want).abs().max().item() <= tol
+            assert (w[m:] == 3).all() and (w[:, n:] == 3).all()
+
+
+def test_the_plan_cuts_where_the_tests_say_so():
+    from speculators_amd.gemm import _tn_list_plan
+
+    cut = {name: _tn_list_plan(tuple((*s, s[1], s[2]) for s in shapes), True)[1] > 0 for name, shapes in LISTS.items()}
+    assert [name for name, is_cut in cut.items() if is_cut] == [name for name in LISTS if "in parts" in name]
+
+
+def test_rules():
+    from speculators_amd import _lib, gemm
+
+    x = torch.zeros(512, 512, dtype=torch.bfloat16, device="cuda")
+    c = torch.zeros(512, 520, device="cuda")
+    good = dict(a=x.data_ptr(), lda=512, b=x.data_ptr(), ldb=512, c=c.data_ptr(), ldc=520, M=512, N=512, T=512)
+    lib, st = _lib.load(), ctypes.c_void_p(_lib.stream_ptr(x.device))
+
+    def rc(n=1, **changes):
+        items = (gemm._TnProduct * 9)(*[gemm._TnProduct(**{**good, **changes})] * 9)
+        return lib.spx_gemm_bf16_tn_list(items, n, 1, None, 0, st)
+
+    assert rc() == 0
+    for changes in ({"T": 128}, {"T": 0}, {"lda": 248, "M": 248}, {"ldb": 516}, {"M": 516}, {"ldc": 504}, {"ldc": 516}, {"a": None},
+                    {"c": c.data_ptr() + 4}, {"n": 0}, {"n": 9}):
+        assert rc(**changes) != 0, changes
+
+
+@pytest.mark.parametrize("regime", ["bf16", "autocast", "mixed"])
+def test_a_layer_staged_together(regime):
+    """The gradients of weights that are staged by one node are those of a node each (the products' sums are the same up to the
+    order of fp32 additions), whichever of them are asked for; nothing is kept alive once the graph is gone."""
+    import gc
+
+    from speculators_amd.gemm import linear_staged
+    from speculators_amd.weights import WeightStager
+
+    torch.manual_seed(1)
+    dt = torch.float32 if regime == "autocast" else torch.bfloat16
+    new = lambda n, k, d=dt: torch.nn.Parameter((torch.randn(n, k, device="cuda") * k ** -0.5).to(d))  # noqa: E731
+    q, k, o, up = new(512, 512), new(256, 512), new(512, 768), new(1024, 512, torch.float32 if regime == "mixed" else dt)
+    x = torch.randn(600, 512, device="cuda").bfloat16()
+
+    def loss(together):
+        stager = WeightStager()
+        stager.begin(uses=2)
+        with torch.autocast("cuda", torch.bfloat16, enabled=regime != "bf16"):
+            if together:
+                wqk, wo, wup = stager.get_all((q, k), (o,), (up,))
+            else:
+                wqk, wo, wup = stager.get(q, k), stager.get(o), stager.get(up)
+            h = x
+            for _ in range(2):
+                h = linear_staged(linear_staged(linear_staged(h, wqk), wo), wup)[:, :512].contiguous()
+        return h.float().square().mean()
+
+    torch.backends.cuda.matmul.allow_bf16_reduced_precision_reduction = False
+    params = (q, k, o, up)
+    want = torch.autograd.grad(loss(False), params)
+    gc.collect()
+    gc.disable()
+    try:
+        before = torch.cuda.memory_allocated()
+        for _ in range(3):
+            got = torch.autograd.grad(loss(True), params)
+            for a, b, p in zip(got, want, params, strict=True):
+                assert a.dtype == p.dtype and (a - b).norm() <= 2 ** -8 * b.norm()
+            del got, a
+        assert torch.cuda.memory_allocated() == before
+        for i, p in enumerate(params):
+            part, = torch.autograd.grad(loss(True), (p,))
+            assert (part - want[i]).norm() <= 2 ** -8 * want[i].norm()
+    finally:
+        gc.enable()

@@ -159,18 +159,20 @@ def test_hand_issued_loads_are_not_read_before_their_wait(tmp_path):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-def test_named_accumulators_are_nobody_elses(tmp_path):
+@pytest.mark.parametrize("source,name,count", [("gemm_bf16_walk.hip", "gemm_bf16_walk_kernel", 6),
+                                               ("gemm_bf16_tn_walk.hip", "gemm_bf16_tn_walk_kernel", 2)])
+def test_named_accumulators_are_nobody_elses(source, name, count, tmp_path):
     """The kernels that walk their tiles hold the accumulators in a0 .. a255 by name: no statement of the compiler's own touches
     an accumulation register, none spills, and around every product lie the issue slots that it needs (as above; a fresh
     product's result has no C operand)."""
-    text = _assembly("gemm_bf16_walk.hip", tmp_path)
+    text = _assembly(source, tmp_path)
 
     def decimal(m):
         return "a[" + ":".join(str(int(x, 0)) for x in m.group(1).split(":")) + "]" if ":" in m.group(1) else f"a{int(m.group(1), 0)}"
 
     text = re.sub(r"\ba\[([\w:]+)\]", decimal, text)
     kernels = 0
-    for m in re.finditer(r"^_ZN3spx21gemm_bf16_walk_kernel\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
+    for m in re.finditer(rf"^_ZN3spx\w*\d{name}\w+:.*?^\.Lfunc_end", text, flags=re.S | re.M):
         kernels += 1
         code, after = _flow(m.group(0).splitlines()[1:-1])
         before = [[] for _ in code]
@@ -197,4 +199,4 @@ def test_named_accumulators_are_nobody_elses(tmp_path):
             _walk(before[n], before, code, 2, ahead)
             _walk(after[n], after, code, 12, behind)
         assert fresh == 64 and sum(p.product for p in code) == 256
-    assert kernels == 6
+    assert kernels == count
