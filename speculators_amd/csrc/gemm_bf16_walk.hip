@@ -26,15 +26,17 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 
 // K: a multiple of 64, at least 192 (and every part of a cut contraction); N and ldc multiples of 8, C 16-byte aligned; SLOW: N a
-// multiple of 256.  m_live, part_ws, max_parts, cus, tail_mode, grade: see gemm_bf16_nt_kernel.
+// multiple of 256.  m_live, part_ws, max_parts, cus, tail_mode, grade: see gemm_bf16_nt_kernel.  parts > 1: all tiles are cut into
+// so many (tail_mode 0), which leave fp32 results in part_ws, [parts][M][N].
 template <bool SLOW, bool GRADE, bool STREAM>
 __global__ __launch_bounds__(kGemmThreads, SPX_GEMM_MINW)
 __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf16_walk_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
     uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K, int tiles_m, int tiles_n,
     const int32_t* __restrict__ m_live, float* __restrict__ part_ws, int max_parts, int cus, int tail_mode,
-    RowGrade grade) {
+    int parts, RowGrade grade) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int M_host = M;
   if (m_live) {
     M = min(M, max(*m_live, 0));
     tiles_m = (M + kTM - 1) / kTM;
@@ -43,6 +45,10 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   int tail_first = n_tiles, tail_parts = 1;
   if (GRADE && tail_mode) live_tail_plan(n_tiles, cus, all_slabs, max_parts, tail_mode, tail_first, tail_parts);
   else if (tail_mode) tail_plan(n_tiles, cus, all_slabs, max_parts, tail_first, tail_parts);
+  if (parts > 1) {
+    tail_first = 0;
+    tail_parts = parts;
+  }
   const int n_tail = n_tiles - tail_first;
   const int n_wg = n_tiles + n_tail * (tail_parts - 1);
   if ((int)blockIdx.x >= n_wg) return;
@@ -76,7 +82,7 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
     if (tail_parts > 1 && pid >= tail_first) {
       const int qq = pid - tail_first, part = small_div(qq, n_tail);
       const int per = (all_slabs + tail_parts - 1) / tail_parts;
-      t.part = qq;  // (part by part, the tiles in their order)
+      t.part = parts > 1 ? part : qq;  // (part by part, the tiles in their order)
       pid = tail_first + qq - part * n_tail;
       k0 = part * per * kTK;
       t.slabs = min(per, all_slabs - part * per);
@@ -247,7 +253,26 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
       at_a = at_b = 0;
     }
     acc.wait();
-    if (cur.part >= 0) {
+    if (cur.part >= 0 && parts > 1) {
+      // this part's fp32 results, in whole lines (rows and columns past the matrix as below)
+      const int cols = min(N - cur.n0, kTN), row_step = N * 64;
+      const u32x4 pres = make_rsrc(part_ws + ((int64_t)cur.part * M_host + cur.m0) * N + cur.n0,
+                                   (uint32_t)((((int64_t)min(M - cur.m0, kTM) - 1) * N + cols) * 4));
+      const bool lo = r16 < 8;
+      const int n = wn + (lo ? 0 : 16) + 4 * q;
+      const int at0 = (int)(((int64_t)(wm + (r16 & 7)) * N + n) * 4);
+      each<kMI * kNI / 2>([&](auto at) __attribute__((always_inline)) {
+        constexpr int i = decltype(at)::value / (kNI / 2), j = decltype(at)::value % (kNI / 2) * 2;
+        u32x4 x, y;
+        const u32x4 v0 = __builtin_bit_cast(u32x4, acc.read<j * kMI + i>());
+        const u32x4 v1 = __builtin_bit_cast(u32x4, acc.read<(j + 1) * kMI + i>());
+        line_pair(lo, v0, v1, x, y);
+        const bool in = n + j * 16 < cols;
+        buffer_store16<j * 64, false>(pres, in ? at0 + i * row_step : kOob, x);
+        buffer_store16<j * 64, false>(pres, in ? at0 + i * row_step + row_step / 2 : kOob, y);
+      });
+      behind = kLB + kMI * kNI;
+    } else if (cur.part >= 0) {
       // this part's fp32 partial of a tile of the last round: a 256 x 256 tile of its own
       float* const P = part_ws + ((int64_t)cur.part << 16) + (wm + r16) * kTN + wn + 4 * q;
       each<kMI * kNI>([&](auto at) __attribute__((always_inline)) {
@@ -297,8 +322,9 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (loads that bring zeros may still be landing in LDS)
 }
 
-bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid) {
-  return K % kTK == 0 && K >= 3 * kTK && N % (slow ? kTN : 8) == 0 && ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0 &&
+bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid, int parts) {
+  const int64_t slabs = K / kTK, per = (slabs + parts - 1) / parts;
+  return K % kTK == 0 && per >= 3 && slabs - per * (parts - 1) >= 3 && (parts == 1 || kTM * N * 4 < 0x7ffffff0ll) && N % (slow ? kTN : 8) == 0 && ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0 &&
          kTM * ldc * 2 < 0x7ffffff0ll && (!slow || (K + 4 * kTK) * ldb * 2 < 0x7ffffff0ll) && n_grid < (1 << 22);
 }
 
@@ -310,12 +336,12 @@ static int launch_walk(const char* fname, const WalkArgs& w, hipStream_t st) {
   hipLaunchKernelGGL((gemm_bf16_walk_kernel<SLOW, GRADE, STREAM>), dim3((unsigned)std::min<int64_t>(w.n_grid, w.cus)),
                      dim3(kGemmThreads), kGemmSmem, st, w.a, w.lda, w.b, w.ldb, w.c, w.ldc, (int)w.M, (int)w.N, (int)w.K,
                      (int)((w.M + kTM - 1) / kTM), (int)((w.N + kTN - 1) / kTN), w.m_live, w.part_ws, w.max_parts, w.cus,
-                     w.tail_mode, w.grade);
+                     w.tail_mode, w.parts, w.grade);
   return check_launch(fname);
 }
 
 int walk(const char* fname, bool slow, const WalkArgs& w, hipStream_t st) {
-  const bool stream = w.M * w.N * 2 > (256ll << 20);
+  const bool stream = w.M * w.N * 2 > (256ll << 20) && w.parts == 1;
   if (slow) return stream ? launch_walk<true, false, true>(fname, w, st) : launch_walk<true, false, false>(fname, w, st);
   if (w.grade.row) return stream ? launch_walk<false, true, true>(fname, w, st) : launch_walk<false, true, false>(fname, w, st);
   return stream ? launch_walk<false, false, true>(fname, w, st) : launch_walk<false, false, false>(fname, w, st);

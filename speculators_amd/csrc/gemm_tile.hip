@@ -247,6 +247,9 @@ static int launch_reduce(const char* fname, const float* ws, void* c, int64_t ld
 // alike; the worst 1.04, 700 x 2048 -> 16384): a b^T 1300 x 8192 -> 6144 184 -> 115 us, 1700 x 5120 -> 5120 115 -> 75,
 // 2900 x 4096 -> 3072 87 -> 63, 3001 x 14336 -> 4096 301 -> 283; a b 1300 x 14336 -> 4096 164 -> 144, 2300 x 4096 -> 4096
 // 90 -> 80, 3001 x 28672 -> 4096 604 -> 556, 5000 x 8192 -> 2048 170 -> 155.
+// The walking kernels (gemm_bf16_walk.hip) and the tiles of three slab buffers of B, fitted again to 136 products of 256 .. 8192 rows
+// (3.6 - 7 % rms): within 0.4 % of the best candidate.  a b, tiles cut whole on the walking kernel, the choice before / now: 1400 x
+// 16384 -> 2048 89 -> 81 us, 3500 rows 186 -> 169, 888 x 28672 -> 4096 186 -> 164, 1100 238 -> 210.
 // (Tiles of 128 x 192 and 256 x 192 are the choice for too few further products, and the slow operand of the second form
 // takes whole powers of two only.)
 enum Tile { kBig = 0, k128x128, k256x128, k64x128, k192x256, kFifth /* NT: 192 x 192, NN: 256 x 256 */, k192x128 /* NN */ };
@@ -254,19 +257,21 @@ struct Config {
   int tm, tn, per_cu;
   float s0, s1, b;
 };
-constexpr Config kNT[] = {{256, 256, 1, 1.18f, 0.23f, 6.9f},   // kBig: gemm_bf16.hip, its last round cut (tail_plan)
+constexpr Config kNT[] = {{256, 256, 1, 0.69f, 0.63f, 6.2f},   // kBig: gemm_bf16_walk.hip, its last round cut (tail_plan)
                           {128, 128, 1, 0.35f, 0.14f, 4.1f},
                           {256, 128, 1, 0.52f, 0.25f, 5.3f},
                           {64, 128, 2, 0.18f, 0.42f, 3.0f},
-                          {192, 256, 1, 1.04f, 0.14f, 8.5f},
-                          {192, 192, 1, 0.61f, 0.23f, 7.0f}};
-constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (no 4-wave kernel of this form)
-                          {128, 128, 1, 0.43f, 0.125f, 0.6f},
-                          {256, 128, 1, 0.59f, 0.22f, 3.9f},
-                          {64, 128, 2, 0.25f, 0.48f, 0.f},
-                          {192, 256, 1, 1.04f, 0.14f, 7.2f},
-                          {256, 256, 1, 1.13f, 0.33f, 4.0f},
-                          {192, 128, 1, 0.50f, 0.14f, 5.5f}};
+                          {192, 256, 1, 0.72f, 0.35f, 6.2f},
+                          {192, 192, 1, 0.53f, 0.28f, 6.0f}};
+// (form 2, rows counted on the device: the large tile as live_tail_plan prices it)
+constexpr Config kLive = {256, 256, 1, 1.18f, 0.23f, 6.9f};
+constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (kFifth)
+                          {128, 128, 1, 0.32f, 0.15f, 3.1f},
+                          {256, 128, 1, 0.55f, 0.25f, 4.8f},
+                          {64, 128, 2, 0.23f, 0.37f, 2.1f},
+                          {192, 256, 1, 0.76f, 0.35f, 5.1f},
+                          {256, 256, 1, 0.78f, 0.47f, 7.4f},   // gemm_bf16_walk.hip
+                          {192, 128, 1, 0.45f, 0.18f, 4.3f}};
 // Weight gradients (contraction slow in both operands): the candidates beside the 256 x 256 kernel of gemm_bf16_tn.hip,
 // which keeps whole rounds of its tiles and is given up only for a predicted tenth.  Fitted the same way to 128 products
 // (results of 1 .. 768 large tiles, 256 .. 20000 rows, up to 12 parts; 6 - 13 % rms).  Over them the choice takes 0.52 of that
@@ -305,7 +310,7 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
   const Config* const table = nn ? kNN : kNT;
   Choice best{kBig, 1, 1e30f};
   if (!nn) {
-    const Config& c = table[kBig];
+    const Config& c = form == 2 ? kLive : table[kBig];
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), rem = tiles % kCus;
     int64_t cut = 0;
     int tp = 1;
@@ -545,13 +550,14 @@ static int auto_product(const char* fname, int form, const void* a, int64_t lda,
   p.part_ws = reinterpret_cast<float*>(workspace);
   p.m_live = m_live;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (form && ch.tile == tile::kFifth && walk_takes(true, c, ldb, ldc, N, K, tiles_m * tiles_n)) {
-    const WalkArgs w = {p.A, lda, p.B, ldb, reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, nullptr, 1, 0, tile::kCus,
-                        tiles_m * tiles_n, RowGrade{}};
-    return walk(fname, true, w, st);
-  }
-  if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st))
+  const int64_t wgs = tiles_m * tiles_n * ch.parts;
+  if (form && ch.tile == tile::kFifth && walk_takes(true, c, ldb, ldc, N, K, wgs, ch.parts)) {
+    const WalkArgs w = {p.A, lda, p.B, ldb, reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, p.part_ws, 1, 0, tile::kCus,
+                        wgs, RowGrade{}, ch.parts};
+    if (int rc = walk(fname, true, w, st)) return rc;
+  } else if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st)) {
     return rc;
+  }
   if (ch.parts == 1) return SPX_OK;
   if (left) {
     *left = ch.parts;

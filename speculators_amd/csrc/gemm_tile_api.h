@@ -39,8 +39,9 @@ struct WalkArgs {
   int max_parts, tail_mode, cus;
   int64_t n_grid;
   RowGrade grade;
+  int parts = 1;  // > 1: the contraction is cut whole, fp32 results in part_ws, [parts][M][N]
 };
-bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid);
+bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid, int parts = 1);
 int walk(const char* fname, bool slow, const WalkArgs& w, hipStream_t st);
 
 namespace tile {

@@ -24,7 +24,10 @@ touches is *staged* once per forward:
     products take it as their differentiable input, and the first one to run its backward
     returns an equally empty marker for it so that the node is reached.  A use whose input
     is not in the buffer (nobody asked for the slot, or it was full) is added by a product of
-    its own (accumulating in fp32);
+    its own (accumulating in fp32).  The weights of a layer are staged by one node
+    (``WeightStager.get_all``), so that their products are one launch.  The nodes hold what the uses
+    left behind (``_Uses``) and not the ``Staged``, whose token leads back to the node: a cycle
+    that Python's collector does not see through where a node has several tokens;
   * frozen weights (``lm_head``, ``verifier_lm_head``, ``embed_tokens``) are
     cast (and transposed where the backward needs it) once and kept until the parameter changes:
     the key is ``(data_ptr, _version, dtype)``; ``WeightStager.invalidate()`` drops every kept

@@ -63,6 +63,23 @@ def test_products_of_workgroups_that_walk(m, n, k, live):
         assert ((matmul_nn(a, b.t().contiguous()).float() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("m,n,k,parts", [(1421, 2048, 16384, 5), (2003, 2048, 16384, 4), (1033, 4096, 28672, 3)])
+def test_walking_products_cut_whole(m, n, k, parts):
+    """The NN product whose every tile is cut along the contraction, the last part the shortest: fp32 partial results of ragged
+    rows, added in their order.  Bound as above; bit for bit the same every time."""
+    from speculators_amd import _lib, gemm
+
+    lib = _lib.load()
+    assert lib.spx_gemm_auto_tile(1, m, n, k, gemm.TAIL_PARTS) == 5
+    assert lib.spx_gemm_auto_workspace_bytes(1, m, n, k, gemm.TAIL_PARTS) == parts * m * n * 4
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a, b = torch.randn(m, k, generator=g, device="cuda").bfloat16(), torch.randn(k, n, generator=g, device="cuda").bfloat16()
+    ref = a.float() @ b.float()
+    got = gemm.matmul_nn(a, b)
+    assert ((got.float() - ref).abs() <= 2 ** -8 * (ref.abs() + k ** 0.5)).all()
+    assert torch.equal(got, gemm.matmul_nn(a, b))
+
+
 def test_gemm_strided_rows():
     from speculators_amd.gemm import gemm_nt
 
