@@ -1267,9 +1267,14 @@ __global__ __launch_bounds__(1024) void mask_row_map_kernel(const void* __restri
 //   of weight zero).
 // TERMS: a weighted sum of kl, ce and tv, as loss_terms_grad_kernel takes it (OP: KL if that is one of them, else CE): a second
 // walk over the registers where tv is a term, and the gradient of the sum.  (rkl and jsd need registers that are not there.)
-// kl, 7 steps of 4096 rows of 32000, 70 % live: a pass a step 1002 us, so 719 (4.7 TB/s; 5.3 for ce: the exponentials of kl
-// take as long as its traffic).  5 steps of 1999 rows without gradient 320 -> 208; {"ce": 0.1, "tv": 0.9}, 3 steps of 3001 407 ->
-// 338.
+// What a step needs of the target row is its probabilities alone (kl: sum p (y - top) once, less sum p (x - top) of each step;
+// the difference is taken thread by thread, before it is added up, and from the row's largest logit on, so that no sum of
+// large terms cancels: mean error against 64 bits 0.97 - 1.03 of that of sum p (y - x), 0 for equal rows either way).  So they
+// are formed once a row and held, in 32 bits: with the draft row's packed chunks 96 of the 128 registers that four waves to a
+// SIMD leave, wherefore chunk numbers are formed again each time.
+// kl, 7 steps of 4096 rows of 32000, 70 % live: a pass a step 1002 us, exponentials of both rows at each step 724, so 663 (5.2
+// TB/s; ce 650, its traffic).  3 steps of 512 rows 52.2 -> 46.0, 7 of 3001 rows of 8192 217 -> 195; 5 of 1999 rows without
+// gradient 199 -> 182, 3 of 333 rows of 1000 with it 16.3 -> 15.1; {"ce": 0.1, "tv": 0.9}, 3 steps of 3001 320 -> 298.
 struct StepsArgs {
   const uint16_t* logits[SPX_LOSS_STEPS_MAX];  // [T, vocab] each
   int64_t ld;
@@ -1297,34 +1302,45 @@ struct StepsArgs {
 
 template <int OP, bool GRAD, bool TERMS = false>
 __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void loss_steps_kernel(StepsArgs a) {
-  constexpr bool kY = OP == SPX_LOSS_KL || TERMS;  // the target row is needed at every step
+  constexpr bool kY = OP == SPX_LOSS_KL || TERMS;  // the target's probabilities are needed at every step
   const int r = blockIdx.x, tid = threadIdx.x, T = a.T;
   const int nchunks = a.vocab >> 3;
   const int rank = GRAD ? a.row_map[r] : -1;
   const bool live = rank >= 0;
   auto row_of = [&](int k) __attribute__((always_inline)) { return r >= k ? r - k : T - k + r; };
+  auto chunk = [&](int j) __attribute__((always_inline)) {  // (formed again each time: held, they would be eight registers)
+    int first = tid;
+    if (kY) asm volatile("" : "+v"(first));
+    return first + j * kFgThreads;
+  };
+  auto at8 = [](const uint16_t* row, int c) __attribute__((always_inline)) {
+    return reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(row) + ((uint32_t)c << 4));
+  };
   auto unpack = [](u32x4 raw, float (&v)[8]) __attribute__((always_inline)) {
     v[0] = bf16_lo(raw.x); v[1] = bf16_hi(raw.x); v[2] = bf16_lo(raw.y); v[3] = bf16_hi(raw.y);
     v[4] = bf16_lo(raw.z); v[5] = bf16_hi(raw.z); v[6] = bf16_lo(raw.w); v[7] = bf16_hi(raw.w);
   };
   u32x4 xr[kFgChunks], yr[kFgChunks];
+  float p[kFgChunks][8];
   const uint16_t* xrow = a.logits[a.k0] + (int64_t)row_of(a.k0) * a.ld;
   const uint16_t* const yrow = a.targets ? a.targets + (int64_t)r * a.ld_targets : nullptr;
   if (a.targets) {
 #pragma unroll
     for (int j = 0; j < kFgChunks; ++j) {
-      const int c = tid + j * kFgThreads;
-      if (c < nchunks) yr[j] = ld16(yrow + ((int64_t)c << 3));
+      if (j * kFgThreads >= nchunks) break;
+      const int c = chunk(j);
+      if (c < nchunks) yr[j] = ld16(at8(yrow, c));
     }
   }
 #pragma unroll
   for (int j = 0; j < kFgChunks; ++j) {
-    const int c = tid + j * kFgThreads;
-    if (c < nchunks) xr[j] = ld16(xrow + ((int64_t)c << 3));
+    if (j * kFgThreads >= nchunks) break;
+    const int c = chunk(j);
+    if (c < nchunks) xr[j] = ld16(at8(xrow, c));
   }
   struct Part { float m, z, a, b; int i; };
   __shared__ Part part[2][kFgWaves];
-  __shared__ float second[2][kFgWaves];
+  __shared__ float second[2][kFgWaves], of_target[kFgThreads];
   int turn = 0;
   // every thread's (maximum, first index of it, sum of 2^(x' - max x'), sum) -> the workgroup's
   auto reduce = [&](float& best, int& at, float& z, float& sum, bool soft) __attribute__((always_inline)) {
@@ -1376,6 +1392,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -m));
   };
 
+  float top = 0.f;  // the target row's largest
   float lt2 = 0.f;  // base-2 log-sum-exp of the target row
   int label;
   if (a.targets) {
@@ -1383,7 +1400,8 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     label = 0x7fffffff;
 #pragma unroll
     for (int j = 0; j < kFgChunks; ++j) {
-      const int c = tid + j * kFgThreads;
+      if (j * kFgThreads >= nchunks) break;
+      const int c = chunk(j);
       if (c >= nchunks) continue;
       float y[8];
       unpack(yr[j], y);
@@ -1392,6 +1410,24 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     }
     reduce(best, label, z, none, kY);
     lt2 = z;
+    top = best;
+    if (kY) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < kFgChunks; ++j) {
+        if (j * kFgThreads >= nchunks) break;
+        if (chunk(j) >= nchunks) continue;
+        asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
+        float y[8];
+        unpack(yr[j], y);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          p[j][i] = fast_exp2(fmaf(y[i], kLog2e, -lt2));
+          sum = fmaf(p[j][i], y[i] - top, sum);
+        }
+      }
+      if (OP == SPX_LOSS_KL) of_target[tid] = sum;
+    }
   } else {
     label = a.argmax_target[r];
     if ((uint32_t)label >= (uint32_t)a.vocab) label = 0;
@@ -1402,11 +1438,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
   for (int k = a.k0; k < a.k1; ++k) {
     const bool tail = r < k;
     const int t = row_of(k);
-    // (nothing of the target row but its packed chunks stays in registers from step to step)
     asm volatile("" : "+v"(label));
-#pragma unroll
-    for (int j = 0; j < kFgChunks; ++j)
-      if (kY) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
     // (a masked row's loss enters no mean: behind the first step it is not formed where gradients are)
     const bool soft = !tail && (!GRAD || live || (k == 0 && a.masked_first));
     const bool more = k + 1 < a.k1;
@@ -1420,41 +1452,40 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     if ((OP == SPX_LOSS_CE || TERMS) && tid == 0) xt = load1(xrow + label);
 #pragma unroll
     for (int j = 0; j < kFgChunks; ++j) {
-      const int c = tid + j * kFgThreads;
+      if (j * kFgThreads >= nchunks) break;
+      const int c = chunk(j);
       if (c >= nchunks) continue;
       float x[8];
       unpack(xr[j], x);
-      if (early) xr[j] = ld16(nrow + ((int64_t)c << 3));
+      if (early) xr[j] = ld16(at8(nrow, c));
       const float cx = largest(x, c << 3, best, at);
       if (soft) {
         soften(x, cx, m, z);
         if (OP == SPX_LOSS_KL) {
-          float y[8];
-          unpack(yr[j], y);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) sum = fmaf(fast_exp2(fmaf(y[i], kLog2e, -lt2)), y[i] - x[i], sum);
+          for (int i = 0; i < 8; ++i) sum = fmaf(p[j][i], x[i] - top, sum);
         }
       }
     }
+    if (OP == SPX_LOSS_KL) sum = of_target[tid] - sum;
     reduce(best, at, z, sum, soft);
     float sum_v = 0.f, ext_v = 0.f;
     if (walk2) {
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {
         asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
-        asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
       }
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {
-        const int c = tid + j * kFgThreads;
+        if (j * kFgThreads >= nchunks) break;
+        const int c = chunk(j);
         if (c >= nchunks) continue;
-        float x[8], y[8];
+        float x[8];
         unpack(xr[j], x);
-        unpack(yr[j], y);
-        if (more && !(GRAD && live)) xr[j] = ld16(nrow + ((int64_t)c << 3));
+        if (more && !(GRAD && live)) xr[j] = ld16(at8(nrow, c));
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const float dp = fast_exp2(fmaf(x[i], kLog2e, -z)), tp = fast_exp2(fmaf(y[i], kLog2e, -lt2));
+          const float dp = fast_exp2(fmaf(x[i], kLog2e, -z)), tp = p[j][i];
           sum_v += fminf(dp, tp);
           ext_v += dp <= tp ? dp : 0.f;
         }
@@ -1495,11 +1526,10 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     }
     if (GRAD && live) {
       uint16_t* const grow = a.grad + ((int64_t)rank * a.steps + k) * a.ld_grad;
-      const float cd = -z, ct = -lt2;
+      const float cd = -z;
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {  // (the packed chunks are what stays in registers between the passes)
         asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
-        if (kY) asm volatile("" : "+v"(yr[j].x), "+v"(yr[j].y), "+v"(yr[j].z), "+v"(yr[j].w));
       }
       // TERMS: every term's gradient is the draft probability times a factor, less w_kl times the target's and w_ce at the label
       const float w_ce = TERMS ? a.tm.w[SPX_LOSS_CE] : 0.f, w_kl = TERMS ? a.tm.w[SPX_LOSS_KL] : 0.f;
@@ -1507,23 +1537,23 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
       const float base_f = w_ce + (OP == SPX_LOSS_KL ? w_kl : 0.f), above = fmaf(w_tv, ext_v, base_f), below = above - w_tv;
 #pragma unroll
       for (int j = 0; j < kFgChunks; ++j) {
-        const int c = tid + j * kFgThreads;
+        if (OP == SPX_LOSS_KL && !TERMS && j * kFgThreads >= nchunks) break;
+        const int c = chunk(j);
         if (c >= nchunks) continue;
         const int base = c << 3;
-        float x[8], y[8], o[8];
+        float x[8], o[8];
         unpack(xr[j], x);
-        if (kY) unpack(yr[j], y);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float dp = fast_exp2(fmaf(x[i], kLog2e, cd));
           if (TERMS) {
-            const float tp = fast_exp2(fmaf(y[i], kLog2e, ct));
+            const float tp = p[j][i];
             o[i] = dp * (dp <= tp ? below : above);
             if (OP == SPX_LOSS_KL) o[i] = fmaf(-w_kl, tp, o[i]);
           } else if (OP == SPX_LOSS_CE) {
             o[i] = dp - ((base + i) == label ? 1.f : 0.f);
           } else {
-            o[i] = dp - fast_exp2(fmaf(y[i], kLog2e, ct));
+            o[i] = dp - p[j][i];
           }
         }
         if (TERMS && c == label >> 3) {
@@ -1534,8 +1564,8 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
           for (int i = 0; i < 8; ++i) o[i] = 0.f;
         }
-        store8_vec<uint16_t>(grow + base, o);
-        if (more) xr[j] = ld16(nrow + base);
+        store8_vec<uint16_t>(const_cast<uint16_t*>(at8(grow, c)), o);
+        if (more) xr[j] = ld16(at8(nrow, c));
       }
     }
     xrow = nrow;

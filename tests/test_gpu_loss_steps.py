@@ -159,3 +159,25 @@ def test_what_goes_step_by_step():
     assert not taken(config=L.resolve_loss_config("jsd")) and not taken(config=L.resolve_loss_config("nla"))
     assert not taken(config={"kl_div": (lambda a, b: a, 1.0)}) and not taken(targets=y.float())
     assert not taken(targets=y[..., 1:], weight=w[1:]) and not taken(targets=y[..., :4088], weight=w[:4088])
+
+
+# (a chunk, a last chunk that a part of one wave holds, all chunks of all threads)
+@pytest.mark.parametrize("vocab", [4096, 4104, 32768])
+@pytest.mark.parametrize("name", ["kl_div", '{"tv": 1.5, "kl_div": 0.25, "ce": 0.125}'])
+def test_target_rows_held_as_probabilities(vocab, name):
+    """Rows that nearly agree, columns of the type's lowest value, and an infinite target: as step by step."""
+    from speculators_amd import losses as L
+
+    config = L.resolve_loss_config(name)
+    x, w, y, mask = _case(50, 3, vocab, 5)
+    y[0] = (x[0][0].float() @ w.float().T).bfloat16()
+    y[0, :, vocab // 2:] = torch.finfo(torch.bfloat16).min
+    want, got = _one_by_one(x, w, y, mask, 0.9, config), _together(x, w, y, mask, 0.9, config)
+    # differences of two log-sum-exps of magnitude <= 16 (ulp 2^-20 at most), each within two units, over three steps
+    assert (got[0] - want[0]).abs() <= 12 * 2.0 ** -20 + 4e-6 * want[0].abs()
+    for a, b in zip(got[4], want[4], strict=True):
+        _close(a, b, 2.0 ** -8)
+    y[0, 25, 3] = -float("inf")
+    mask[0, 25] = 1
+    want, got = _one_by_one(x, w, y, mask, 0.9, config), _together(x, w, y, mask, 0.9, config)
+    assert torch.equal(got[0].isnan(), want[0].isnan())
