@@ -384,8 +384,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, weight_t: torch.Tensor | None 
 
 # Which GEMM runs the decoder-layer projections (q/k/v, o, gate/up, down and their input
 # gradients): "hipblaslt" = PyTorch's matmul (the library GEMM), "spx" = this library's MFMA kernels, "mixed" =
-# each where it is faster: the forward products as ``_own_forward`` says, the input gradients on this library's
-# kernels (``input_gradient``: on the weight as it lies, or on its transposed copy).  The fc / lm_head /
+# each where it is faster: the forward products as ``_own_forward`` and ``_walking_forward`` say, the input gradients on
+# this library's kernels (``input_gradient``: on the weight as it lies, or on its transposed copy).  The fc / lm_head /
 # verifier-head products and every weight gradient always run on this library's kernels.
 DECODER_GEMM = os.environ.get("SPX_DECODER_GEMM", "mixed")
 if DECODER_GEMM not in ("hipblaslt", "spx", "mixed"):
@@ -427,12 +427,37 @@ def _own_forward(m: int, n: int, k: int) -> bool:
     return _on_192_rows(m, n, k, TAIL_PARTS)
 
 
+@functools.lru_cache(maxsize=4096)
+def _walking_forward(m: int, n: int, k: int) -> bool:
+    """Of what ``_own_forward`` leaves to the library, the products that workgroups which walk the large tiles take as fast or
+    faster (ratios: own time to hipBLASLt's, 156 products of 700 to 32760 rows of the 1B, 8B and 70B shapes and others; each is a
+    library call of some 25 us on the host less, too).
+
+    Contractions below 4096: 0.71 - 1.02 over 52 products, 0.95 in the geometric mean (1B gate/up 0.96 - 1.02, its results
+    leave under the next tile's loads).  A last round cut along the contraction: 0.65 - 1.01 over 22 (0.86; 8B gate/up 0.77 -
+    1.01, 70B gate/up 0.90 - 0.93).  Contractions from 16384 on: 0.64 - 1.02 over 22 (0.86).  Left to the library: whole
+    rounds over 4096 to 16383, 0.84 - 1.05 over 55 (1.00, but 1.01 - 1.05 where N is a power of two or three of them), and
+    the tiles of 192 rows."""
+    if not m or k % 64 or n % 8 or _lib.load().spx_gemm_auto_tile(0, m, n, k, TAIL_PARTS):
+        return False
+    if k < 4096:
+        return True
+    return m > 1024 and (k >= 16384 or _forward_route("spx", TAIL_PARTS, m, n, k)[0] == TAIL)
+
+
+def _rows_in_lines(t: torch.Tensor) -> bool:
+    """Whether the 256 x 256 kernels read a matrix as it lies."""
+    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.shape[1] <= t.stride(0) < 1 << 21 and t.data_ptr() % 16 == 0
+
+
 def _project(x2: torch.Tensor, staged) -> torch.Tensor:
     """``x2 @ staged.w.T`` of a decoder-layer projection."""
     if DECODER_GEMM == "spx":
         return matmul_nt(x2, staged.w)
-    if DECODER_GEMM == "mixed" and x2.dtype == torch.bfloat16 and _own_forward(x2.shape[0], *staged.w.shape):
-        return matmul_nt(x2, staged.w)
+    if DECODER_GEMM == "mixed" and x2.dtype == torch.bfloat16:
+        m, (n, k) = x2.shape[0], staged.w.shape
+        if _own_forward(m, n, k) or (_walking_forward(m, n, k) and _rows_in_lines(x2) and _rows_in_lines(staged.w)):
+            return matmul_nt(x2, staged.w)
     return torch.nn.functional.linear(x2, staged.w)
 
 
@@ -446,9 +471,9 @@ def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
 
 
 @functools.lru_cache(maxsize=4096)
-def _forward_route(mode: str, parts: int, m: int, n: int, k: int):
-    """``(route, workspace elements)`` of ``_project`` for contiguous rows."""
-    if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k)):
+def _forward_route(mode: str, parts: int, m: int, n: int, k: int, lines: bool = True):
+    """``(route, workspace elements)`` of ``_project`` for contiguous rows (``lines``: of a weight of ``_rows_in_lines``)."""
+    if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k) and not (lines and _walking_forward(m, n, k))):
         return LINEAR, 0
     big, ws_numel, _ = _plan(0, m, n, k, parts)
     if not big and k % 8 == 0:
@@ -460,7 +485,7 @@ def _forward_route(mode: str, parts: int, m: int, n: int, k: int):
 
 
 def forward_route(m: int, staged):
-    return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *staged.w.shape)
+    return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *staged.w.shape, _rows_in_lines(staged.w))
 
 
 @functools.lru_cache(maxsize=4096)

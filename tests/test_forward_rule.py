@@ -25,3 +25,15 @@ def test_nothing_that_ran_here_without_the_tall_tiles_goes_to_the_library():
         tile = _lib.load().spx_gemm_auto_tile(2, m, n, k, gemm.TAIL_PARTS)  # the choice without tiles of 192 rows
         if tile and m <= 1024:
             assert gemm._own_forward(m, n, k), (m, n, k)
+
+
+@pytest.mark.parametrize("rows,n,k,here", [
+    # short contractions, a cut last round, long contractions; whole rounds between stay with the library, as do no rows and
+    # sizes that workgroups do not walk
+    (888, 16384, 2048, True), (32760, 12288, 2048, True), (3001, 28672, 4096, True), (5000, 6144, 16384, True),
+    (4096, 28672, 4096, False), (888, 28672, 4096, False), (0, 16384, 2048, False), (3001, 16384, 2080, False),
+    (3001, 16380, 2048, False)])
+def test_products_that_workgroups_walk(rows, n, k, here):
+    assert not gemm._own_forward(rows, n, k) and gemm._walking_forward(rows, n, k) == here
+    assert (gemm._forward_route("mixed", gemm.TAIL_PARTS, rows, n, k)[0] != gemm.LINEAR) == here
+    assert gemm._forward_route("mixed", gemm.TAIL_PARTS, rows, n, k, False)[0] == gemm.LINEAR
