@@ -159,6 +159,8 @@ SIGNATURES["spx_gemm_auto_tile"] = [_I, _I64, _I64, _I64, _I32]
 SIGNATURES["spx_gemm_graded_workspace_bytes"] = [_I64, _I64, _I64, _I32, _I32]
 SIGNATURES["spx_gemm_graded_parts"] = [_I64, _I64, _I64, _I32, _I32, _I64, _I64]
 SIGNATURES["spx_gemm_bf16_auto_parts"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P]
+SIGNATURES["spx_gemm_pair_takes"] = [_I, _I64, _I64, _I64, _I64, _I32]
+SIGNATURES["spx_gemm_bf16_pair"] = [_I, _P, _I64, _P, _P, _I64, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P]
 SIGNATURES["spx_gemm_bf16_auto"] = [_I, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P]
 SIGNATURES["spx_stage_upload"] = [_P, _I64, _P, _P, _I64, _I32, _P]
 RESTYPES = {"spx_gemm_auto_workspace_bytes": c_int64, "spx_gemm_graded_workspace_bytes": c_int64, "spx_gemm_tn_workspace_bytes": c_int64, "spx_gemm_auto_us": c_float, "spx_gemm_tn_us": c_float, "spx_gemm_tn_list_us": c_float, "spx_gemm_tn_list_workspace_bytes": c_int64, "spx_moe_sort_workspace_bytes": c_int64, "spx_loss_steps_partials": c_int64, "spx_gemm_grouped_workspace_bytes": c_int64, "spx_gemm_tail_workspace_bytes": c_int64, "spx_gemm_stats_workspace_bytes": c_int64, "spx_gemm_split_workspace_bytes": c_int64, "spx_ttt_attn_workspace_bytes": c_int64, "spx_ttt_attn_fwd_static_max_bytes": c_int64, "spx_dflash_attn_workspace_bytes": c_int64,

@@ -622,7 +622,7 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
                         const int32_t* tile_tab = nullptr, const int32_t* group_off = nullptr,
                         int64_t b_group_stride = 0, int64_t groups = 0, float* part_ws = nullptr,
                         int max_parts = 1, float* stat_ws = nullptr, int stats_mode = 0, int tail_mode = 0,
-                        const RowGrade& grade = RowGrade{}) {
+                        const RowGrade& grade = RowGrade{}, const void* b2 = nullptr) {
   SPX_REQ_FN(M > 0 && N > 0 && K > 0, "M, N, K must be positive");
   SPX_REQ_FN(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "dimension too large");
   SPX_REQ_FN(a && b && (c || stat_ws), "null buffer");
@@ -665,9 +665,11 @@ static int gemm_nt_impl(const char* fname, const void* a, int64_t lda, const voi
   // (row statistics, groups and products that are cut whole have a workgroup a tile)
   if (!stat_ws && !tile_tab && (!part_ws || tail_mode) && walk_takes(false, c, ldb, ldc, N, K, n_grid)) {
     const WalkArgs w = {reinterpret_cast<const uint16_t*>(a), lda, reinterpret_cast<const uint16_t*>(b), ldb,
-                        reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, part_ws, max_parts, tail_mode, cus, n_grid, grade};
+                        reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, part_ws, max_parts, tail_mode, cus, n_grid, grade, 1,
+                        reinterpret_cast<const uint16_t*>(b2)};
     if (int rc = walk(fname, false, w, st)) return rc;
   } else {
+    SPX_REQ_FN(!b2, "a second half of b: sizes that workgroups walk");
     if (int rc = ensure_dynamic_lds(fns[which], kGemmSmem, lds_set[which], fname)) return rc;
 #define SPX_GEMM_LAUNCH(IMM, ...)                                                                                \
   hipLaunchKernelGGL((gemm_bf16_nt_kernel<IMM, __VA_ARGS__>), grid, block, kGemmSmem, st,                        \
@@ -797,6 +799,12 @@ extern "C" int spx_gemm_bf16_nt_tail(const void* a, int64_t lda, const void* b, 
   SPX_REQ_FN(workspace_bytes >= spx_gemm_tail_workspace_bytes(), "workspace too small");
   return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, nullptr, stream, nullptr, nullptr, 0, 0,
                       reinterpret_cast<float*>(workspace), max_parts, nullptr, 0, 1);
+}
+
+int spx::nt_pair(const char* fname, const void* a, int64_t lda, const void* b, const void* b2, int64_t ldb, void* c, int64_t ldc,
+                 int64_t M, int64_t N, int64_t K, float* part_ws, int max_parts, void* stream) {
+  return gemm_nt_impl(fname, a, lda, b, ldb, c, ldc, M, N, K, nullptr, stream, nullptr, nullptr, 0, 0, part_ws, part_ws ? max_parts : 1,
+                      nullptr, 0, part_ws ? 1 : 0, RowGrade{}, b2);
 }
 
 extern "C" int64_t spx_gemm_stats_workspace_bytes(int64_t M, int64_t N) {

@@ -28,11 +28,15 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 // K: a multiple of 64, at least 192 (and every part of a cut contraction); N and ldc multiples of 8, C 16-byte aligned; SLOW: N a
 // multiple of 256.  m_live, part_ws, max_parts, cus, tail_mode, grade: see gemm_bf16_nt_kernel.  parts > 1: all tiles are cut into
 // so many (tail_mode 0), which leave fp32 results in part_ws, [parts][M][N].
+// B2 (else null): the second half of B's rows -- its first `half` rows are at B, the others at B2, both ldb apart.  A tile of the
+// plain form lies in one of them (half % 256 == 0); SLOW: the loads turn to B2 with the slab that starts there (half % 64 == 0),
+// which is never the second or third of a tile or of a part of one.  (Asked for at every slab instead of where it comes, the turn
+// cost all products of that form 0.5 - 1.4 %.)
 template <bool SLOW, bool GRADE, bool STREAM>
 __global__ __launch_bounds__(kGemmThreads, SPX_GEMM_MINW)
 __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf16_walk_kernel(
-    const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
-    uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K, int tiles_m, int tiles_n,
+    const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, const uint16_t* __restrict__ B2, int half,
+    int64_t ldb, uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K, int tiles_m, int tiles_n,
     const int32_t* __restrict__ m_live, float* __restrict__ part_ws, int max_parts, int cus, int tail_mode,
     int parts, RowGrade grade) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -56,12 +60,14 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   struct Tile {
     int m0, n0, slabs, part;  // part: of a tile that is cut, its place in part_ws, else -1
     u32x4 ares, bres;
+    int turn;  // SLOW: slabs until B2
   };
   auto tile_at = [&](int id) __attribute__((always_inline)) {
     Tile t;
     if (id >= n_wg) {  // nothing: its loads bring zeros
       t.m0 = t.n0 = t.slabs = 0;
       t.part = -1;
+      t.turn = 0x7fffffff;
       t.ares = make_rsrc(A, 0);
       t.bres = make_rsrc(B, 0);
       return t;
@@ -93,10 +99,14 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
     t.n0 = tile_n * kTN;
     // (rows past the matrix lie outside the resource: they are lda, ldb >= K apart)
     t.ares = make_rsrc(A + (int64_t)t.m0 * lda + k0, (uint32_t)((((int64_t)min(M - t.m0, kTM) - 1) * lda + K - k0) * 2));
+    const int at = SLOW ? k0 : t.n0;  // the first row of B
+    const bool second = B2 && at >= half;
+    const uint16_t* const rows = second ? B2 + (int64_t)(at - half) * ldb : B + (int64_t)at * ldb;
+    t.turn = !SLOW || !B2 || second ? 0x7fffffff : (half - k0) / kTK;
     if (SLOW)
-      t.bres = make_rsrc(B + (int64_t)k0 * ldb + t.n0, (uint32_t)((((int64_t)K - k0 - 1) * ldb + kTN) * 2));
+      t.bres = make_rsrc(rows + t.n0, (uint32_t)((((int64_t)(B2 && !second ? half : K) - k0 - 1) * ldb + kTN) * 2));
     else
-      t.bres = make_rsrc(B + (int64_t)t.n0 * ldb + k0, (uint32_t)((((int64_t)min(N - t.n0, kTN) - 1) * ldb + K - k0) * 2));
+      t.bres = make_rsrc(rows + k0, (uint32_t)((((int64_t)min(N - t.n0, kTN) - 1) * ldb + K - k0) * 2));
     return t;
   };
 
@@ -245,9 +255,16 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
     const Tile next = tile_at(id);
     slab(std::true_type{}, behind);
     int s = 1;
-    for (int end = cur.slabs - 2;; end = cur.slabs) {
+    for (int end = (SLOW && cur.turn < cur.slabs ? cur.turn : cur.slabs) - 2;;) {  // (the loads are two slabs ahead)
       for (; s < end; ++s) slab(std::false_type{}, kLB);
       if (end == cur.slabs) break;
+      if (SLOW && end != cur.slabs - 2) {
+        bres = make_rsrc(B2 + cur.n0, (uint32_t)((((int64_t)K - half - 1) * ldb + kTN) * 2));
+        at_b = 0;
+        end = cur.slabs - 2;
+        continue;
+      }
+      end = cur.slabs;
       ares = next.ares;
       bres = next.bres;
       at_a = at_b = 0;
@@ -334,7 +351,8 @@ static int launch_walk(const char* fname, const WalkArgs& w, hipStream_t st) {
   auto* const kernel = &gemm_bf16_walk_kernel<SLOW, GRADE, STREAM>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kGemmSmem, lds_set, fname)) return rc;
   hipLaunchKernelGGL((gemm_bf16_walk_kernel<SLOW, GRADE, STREAM>), dim3((unsigned)std::min<int64_t>(w.n_grid, w.cus)),
-                     dim3(kGemmThreads), kGemmSmem, st, w.a, w.lda, w.b, w.ldb, w.c, w.ldc, (int)w.M, (int)w.N, (int)w.K,
+                     dim3(kGemmThreads), kGemmSmem, st, w.a, w.lda, w.b, w.b2, w.b2 ? (int)((SLOW ? w.K : w.N) / 2) : 0,
+                     w.ldb, w.c, w.ldc, (int)w.M, (int)w.N, (int)w.K,
                      (int)((w.M + kTM - 1) / kTM), (int)((w.N + kTN - 1) / kTN), w.m_live, w.part_ws, w.max_parts, w.cus,
                      w.tail_mode, w.parts, w.grade);
   return check_launch(fname);

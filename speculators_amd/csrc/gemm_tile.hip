@@ -522,7 +522,7 @@ extern "C" int spx_gemm_auto_tile(int form, int64_t M, int64_t N, int64_t K, int
 // left: where the number of partial results goes that are left in the workspace (NULL: they are added here)
 static int auto_product(const char* fname, int form, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                         int64_t ldc, int64_t M, int64_t N, int64_t K, const int32_t* m_live, int32_t max_parts,
-                        void* workspace, int64_t workspace_bytes, int32_t* left, void* stream) {
+                        void* workspace, int64_t workspace_bytes, int32_t* left, void* stream, const void* b2 = nullptr) {
   if (left) *left = 1;
   SPX_REQ_FN(max_parts >= 1 && max_parts <= 8, "max_parts must be 1 .. 8");
   if (int rc = tile::dense_check(fname, form, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
@@ -553,7 +553,7 @@ static int auto_product(const char* fname, int form, const void* a, int64_t lda,
   const int64_t wgs = tiles_m * tiles_n * ch.parts;
   if (form && ch.tile == tile::kFifth && walk_takes(true, c, ldb, ldc, N, K, wgs, ch.parts)) {
     const WalkArgs w = {p.A, lda, p.B, ldb, reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, p.part_ws, 1, 0, tile::kCus,
-                        wgs, RowGrade{}, ch.parts};
+                        wgs, RowGrade{}, ch.parts, reinterpret_cast<const uint16_t*>(b2)};
     if (int rc = walk(fname, true, w, st)) return rc;
   } else if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st)) {
     return rc;
@@ -580,6 +580,37 @@ extern "C" int spx_gemm_bf16_auto_parts(int form, const void* a, int64_t lda, co
   SPX_REQ_FN(parts, "null buffer");
   return auto_product(fname, form, a, lda, b, ldb, c, ldc, M, N, K, nullptr, max_parts, workspace, workspace_bytes, parts,
                       stream);
+}
+
+extern "C" int spx_gemm_pair_takes(int form, int64_t M, int64_t N, int64_t K, int64_t ldb, int32_t max_parts) {
+  if ((form != 0 && form != 1) || M <= 0 || N <= 0 || K <= 0 || ldb < (form ? N : K) || ldb % 8 || max_parts < 1 || max_parts > 8) return 0;
+  const int64_t half = (form ? K : N) / 2;
+  if (half * 2 != (form ? K : N) || half % (form ? 64 : 256)) return 0;
+  const tile::Choice ch = tile::choose(form, M, N, K, max_parts, can_split(N));
+  const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256);
+  if (ch.tile != (form ? tile::kFifth : tile::kBig)) return 0;
+  if (form) {  // (a part's first two slabs lie in the same half: they are requested before its tile is turned to)
+    const int64_t slabs = K / 64, per = (slabs + ch.parts - 1) / ch.parts, before = slabs / 2 % per;
+    if (before == 1 || before == 2) return 0;
+  }
+  return walk_takes(form == 1, nullptr, ldb, N, N, K, tiles + (form ? tiles * (ch.parts - 1) : 8 * tile::kCus), form ? ch.parts : 1);
+}
+
+extern "C" int spx_gemm_bf16_pair(int form, const void* a, int64_t lda, const void* b, const void* b2, int64_t ldb, void* c, int64_t ldc,
+                                  int64_t M, int64_t N, int64_t K, int32_t max_parts, void* workspace, int64_t workspace_bytes,
+                                  int32_t* parts, void* stream) {
+  const char* fname = __func__;
+  if (parts) *parts = 1;
+  if (int rc = tile::dense_check(fname, form, a, lda, b, ldb, c, ldc, M, N, K)) return rc;
+  SPX_REQ_FN(b2 && ((uintptr_t)b2) % 16 == 0, "null or unaligned second half");
+  SPX_REQ_FN(ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0, "ldc must be a multiple of 8 and c 16-byte aligned");
+  SPX_REQ_FN(spx_gemm_pair_takes(form, M, N, K, ldb, max_parts) && 256 * ldc * 2 < 0x7ffffff0ll, "sizes that spx_gemm_pair_takes refuses");
+  if (form) {
+    SPX_REQ_FN(workspace_bytes >= spx_gemm_auto_workspace_bytes(1, M, N, K, max_parts), "workspace too small");
+    return auto_product(fname, 1, a, lda, b, ldb, c, ldc, M, N, K, nullptr, max_parts, workspace, workspace_bytes, parts, stream, b2);
+  }
+  const bool cut = max_parts > 1 && workspace && ((uintptr_t)workspace) % 16 == 0 && workspace_bytes >= spx_gemm_tail_workspace_bytes();
+  return nt_pair(fname, a, lda, b, b2, ldb, c, ldc, M, N, K, cut ? reinterpret_cast<float*>(workspace) : nullptr, max_parts, stream);
 }
 
 // The weights in the product's own epilogue (a load per row and a multiply per result) or in the pass that adds its parts; the

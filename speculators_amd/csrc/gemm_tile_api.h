@@ -40,9 +40,15 @@ struct WalkArgs {
   int64_t n_grid;
   RowGrade grade;
   int parts = 1;  // > 1: the contraction is cut whole, fp32 results in part_ws, [parts][M][N]
+  const uint16_t* b2 = nullptr;  // the second half of b's rows (half of N, slow: of K), where they are not behind the first
 };
 bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid, int parts = 1);
 int walk(const char* fname, bool slow, const WalkArgs& w, hipStream_t st);
+
+// a b^T of the 256 x 256 kernels, its last round cut where there is part_ws, b's second half of rows at b2 (gemm_bf16.hip); the sizes
+// are what walk_takes says
+int nt_pair(const char* fname, const void* a, int64_t lda, const void* b, const void* b2, int64_t ldb, void* c, int64_t ldc, int64_t M,
+            int64_t N, int64_t K, float* part_ws, int max_parts, void* stream);
 
 namespace tile {
 

@@ -112,7 +112,7 @@ void norm_backward(const Tensor& x, const Tensor& gain, const Parted& dy, const 
 }
 
 // How gemm.py routed a product (``Route`` there)
-enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul };
+enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul, kPairNT, kPairNN };
 struct Products {
   int64_t parts;
   Tensor ws;  // fp32 partials of products cut along the contraction
@@ -134,6 +134,18 @@ struct Products {
       check(spx_gemm_bf16_auto(route, in(a), a.stride(0), in(b), b.stride(0), to(out), n, m, n, k,
                                m_live.defined() ? m_live.const_data_ptr<int32_t>() : nullptr, parts, w, wb, st),
             "spx_gemm_bf16_auto");
+    return out;
+  }
+  // the rows of b in two matrices (kPairNT, kPairNN); count: as Parted, null where the result is to be stored
+  Tensor pair(int64_t route, const Tensor& a, const Tensor& b, const Tensor& b2, int32_t* count = nullptr) const {
+    const bool nn = route == kPairNN;
+    const int64_t m = a.size(0), k = a.size(1), n = nn ? b.size(1) : 2 * b.size(0);
+    TORCH_CHECK_VALUE(b2.defined() && b2.sizes() == b.sizes() && b2.stride(0) == b.stride(0) && (nn ? 2 * b.size(0) : b.size(1)) == k,
+                      "shape mismatch: a ", a.sizes(), " and two of b ", b.sizes());
+    const Tensor out = at::empty({m, n}, a.options());
+    check(spx_gemm_bf16_pair(nn, in(a), a.stride(0), in(b), in(b2), b.stride(0), to(out), n, m, n, k, parts,
+                             ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, count, stream_of(a)),
+          "spx_gemm_bf16_pair");
     return out;
   }
   // for a launch that adds the parts of a cut product itself
@@ -167,22 +179,23 @@ PyObject* spx_layer_product(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // Behind the attention: o, residual add + norm, gate/up, SwiGLU, down, residual add + the next norm.
 PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Args x("tail_forward", args, n, 17);
+  Args x("tail_forward", args, n, 18);
   const Tensor &residual = x.tensor(), &att = x.tensor(), &wo = x.tensor(), &wgu = x.tensor(), &wd = x.tensor(),
                &gain_post = x.tensor(), &gain_next = x.tensor(), slot_gu = x.maybe(), slot_d = x.maybe(),
                slot_next = x.maybe();
   const double eps_post = x.number(), eps_next = x.number();
   const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
+  const Tensor wu = x.maybe();  // r_gu kPairNT: wgu is gate's alone
   Unlocked released;
-  const int64_t t = residual.size(0), h = residual.size(1), f = wgu.size(0) / 2;
+  const int64_t t = residual.size(0), h = residual.size(1), f = r_gu == kPairNT ? wgu.size(0) : wgu.size(0) / 2;
   void* const st = stream_of(residual);
   const Tensor stats = at::empty({2, t}, residual.options().dtype(at::kFloat));
   float* const rstd = floats(stats);
   const Parted o = product.parted(r_o, att, wo);
   const Tensor mid = at::empty({t, h}, residual.options()), z = rows_or_new(slot_gu, t, h, residual);
   add_norm(residual, o, mid, gain_post, z, rstd, eps_post, st);
-  const Tensor gu = product(r_gu, z, wgu), act = rows_or_new(slot_d, t, f, residual);
+  const Tensor gu = r_gu == kPairNT ? product.pair(r_gu, z, wgu, wu) : product(r_gu, z, wgu), act = rows_or_new(slot_d, t, f, residual);
   check(spx_swiglu_rows_fwd(in(gu), 2 * f, in(gu) + f, 2 * f, to(act), f, t, f, st), "spx_swiglu_rows_fwd");
   const Parted m = product.parted(r_d, act, wd);
   const Tensor y = at::empty({t, h}, residual.options()), normed = rows_or_new(slot_next, t, h, residual);
@@ -195,7 +208,7 @@ PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n)
 // partial sums of the gains' gradients (accumulate: added to).
 PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Args x("tail_backward", args, n, 23);
+  Args x("tail_backward", args, n, 24);
   const Tensor dy = x.maybe(), dn = x.maybe();
   const Tensor &mid = x.tensor(), &stats = x.tensor(), &gu = x.tensor(), &y = x.tensor(), &gain_post = x.tensor(),
                &gain_next = x.tensor(), &bo = x.tensor(), &bgu = x.tensor(), &bd = x.tensor(), slot_d = x.maybe(),
@@ -205,6 +218,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   const int64_t acc_next = x.integer();
   const int64_t r_o = x.integer(), r_gu = x.integer(), r_d = x.integer(), parts = x.integer();
   const Products product{parts, x.maybe()};
+  const Tensor bu = x.maybe();  // r_gu kPairNN: bgu is gate's alone
   Unlocked released;
   const int64_t t = y.size(0), h = y.size(1), f = gu.size(1) / 2;
   void* const st = stream_of(y);
@@ -219,7 +233,13 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
   const Tensor dact = product(r_d, dm, bd), dgu = rows_or_new(slot_gu, t, 2 * f, y);
   check(spx_swiglu_rows_bwd(in(gu), 2 * f, in(gu) + f, 2 * f, in(dact), f, to(dgu), 2 * f, to(dgu) + f, 2 * f, t, f, st),
         "spx_swiglu_rows_bwd");
-  const Parted dz = product.parted(r_gu, dgu, bgu);
+  Parted dz;
+  if (r_gu == kPairNN) {
+    dz.stored = product.pair(r_gu, dgu, bgu, bu, product.ws.defined() ? &dz.count : nullptr);
+    if (dz.count > 1) dz.at = product.ws.const_data_ptr<float>();
+  } else {
+    dz = product.parted(r_gu, dgu, bgu);
+  }
   const Tensor da = rows_or_new(slot_o, t, h, y);
   norm_backward(mid, gain_post, dz, dm, rstd, da, scratch_post, acc_post, st);
   return tuple_of(released, {dm, dgu, da, product(r_o, da, bo)});

@@ -135,7 +135,7 @@ def _graded_workspace(m: int, n: int, k: int, parts: int, split: int) -> int:
 
 # how a product runs, as csrc/layer_host.cpp numbers it: on spx_gemm_bf16_auto (NT or NN form), on the 256 x 256 kernel
 # without or with its last round cut, or in the library
-AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL = range(6)
+AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL, PAIR_NT, PAIR_NN = range(8)
 
 
 def _auto(form: int, a, b, ws_numel: int, m_live=None):
@@ -207,7 +207,7 @@ def input_gradient(dy2: torch.Tensor, staged) -> torch.Tensor:
     weight's uses; that of a frozen weight is kept."""
     if _nn_fits(dy2, staged.w):
         m, (k, n) = dy2.shape[0], staged.w.shape
-        copy_us = 0.0 if staged.has_wt or not staged.trainable else (3.0 + _TRANSPOSE_US * 1e-6 * k * n) / staged.uses
+        copy_us = 0.0 if staged.has_wt or not staged.trainable else _copy_us(k, n, staged.uses)
         if _plan(1, m, n, k, TAIL_PARTS)[2] <= _plan(0, m, n, k, TAIL_PARTS)[2] + copy_us:
             return matmul_nn(dy2, staged.w)
     return matmul_nt(dy2, staged.wt)
@@ -500,14 +500,50 @@ def _backward_route(mode: str, parts: int, m: int, k: int, n: int, ld: int, alig
     return (*_forward_route("spx", parts, m, n, k), True)
 
 
+def _copy_us(k: int, n: int, uses: int) -> float:
+    """What the transposed copy of a weight costs each of its uses."""
+    return (3.0 + _TRANSPOSE_US * 1e-6 * k * n) / uses
+
+
 def backward_route(m: int, staged):
     """``(route, workspace elements, right operand)`` of the input gradient of a product with ``m`` rows."""
     w = staged.w
     k, n = w.shape
-    copy_us = 0.0 if staged.has_wt or not staged.trainable else (3.0 + _TRANSPOSE_US * 1e-6 * k * n) / staged.uses
+    copy_us = 0.0 if staged.has_wt or not staged.trainable else _copy_us(k, n, staged.uses)
     route, ws, transposed = _backward_route(DECODER_GEMM, TAIL_PARTS, m, k, n, w.stride(0), w.data_ptr() % 16 == 0,
                                             copy_us)
     return route, ws, staged.wt if transposed else w
+
+
+@functools.lru_cache(maxsize=4096)
+def _pair_routes(mode: str, parts: int, m: int, f: int, h: int, trainable: bool, uses: int):
+    """See ``pair_routes``.
+
+    The concatenation that falls away reads and writes 4 f h bytes at 5 TB/s once a forward (8B shape 94 us, 1B 22 us; the products
+    themselves take the same time, within 0.7 %: a validation pass of the 1B shape 1.013, the anchored-block draft of the 8B shape
+    54.16 -> 53.97 ms).  A product that would run on the library otherwise may take 4 % longer for it, at every use; the input
+    gradient has to be one that is formed on the weight as it lies, by workgroups that walk the tiles."""
+    lib = _lib.load()
+    if mode == "hipblaslt" or m <= 0 or not lib.spx_gemm_pair_takes(0, m, 2 * f, h, h, parts):
+        return None
+    route, ws = _forward_route("spx", parts, m, 2 * f, h)
+    if mode == "mixed" and _forward_route(mode, parts, m, 2 * f, h)[0] == LINEAR \
+            and 0.04 * _plan(0, m, 2 * f, h, parts)[2] * uses > 8e-6 * f * h / 5:
+        return None
+    if not trainable:
+        return ws, 0
+    if not lib.spx_gemm_pair_takes(1, m, h, 2 * f, h, parts) \
+            or _plan(1, m, h, 2 * f, parts)[2] > _plan(0, m, h, 2 * f, parts)[2] + _copy_us(2 * f, h, uses):
+        return None
+    return ws, _plan(1, m, h, 2 * f, parts)[1]
+
+
+def pair_routes(m: int, staged):
+    """Whether the products with ``m`` rows against a weight of two parameters take these as they lie (``spx_gemm_bf16_pair``): the
+    workspace elements of the forward product and of the input gradient, else None (they take ``staged.w``)."""
+    if staged.pieces is None:
+        return None
+    return _pair_routes(DECODER_GEMM, TAIL_PARTS, m, *staged.pieces[0].shape, staged.trainable, staged.uses)
 
 
 def workspace_for(device, *numels):

@@ -42,7 +42,7 @@ class LayerStep:
     """What a step needs besides its differentiable inputs."""
 
     __slots__ = ("first", "wqkv", "wo", "wgu", "wd", "eps_in", "eps_post", "eps_next", "hq", "hkv", "d", "scaling",
-                 "offset", "positions", "inv_freq", "cache", "mask", "slots")
+                 "offset", "positions", "inv_freq", "cache", "mask", "slots", "pair")
 
     def __init__(self, first, wqkv, wo, wgu, wd, eps, heads, scaling, offset, positions, inv_freq, cache, mask):
         self.first = first
@@ -61,7 +61,12 @@ class LayerStep:
 
     def constants(self):
         """What the backward reads beside activations and gains, to be saved with the node."""
-        return (self.positions, self.inv_freq, self.mask.row_lo, self.wqkv.w, self.wo.w, self.wgu.w, self.wd.w)
+        return (self.positions, self.inv_freq, self.mask.row_lo, self.wqkv.w, self.wo.w, self.wd.w, *_gate_up(self))
+
+
+def _gate_up(s):
+    """The weight of the gate and up projections as the products read it."""
+    return (s.wgu.w,) if s.pair is None else s.wgu.pieces
 
 
 def _rows(t, rows, cols, device):
@@ -100,10 +105,14 @@ def _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_
     """What follows the attention: output projection, residual add and norm, MLP, residual add and the norm
     that reads the layer's output."""
     t = residual.shape[0]
-    routes, sizes = zip(*(gemm.forward_route(t, w) for w in (s.wo, s.wgu, s.wd)))
+    s.pair = gemm.pair_routes(t, s.wgu)
+    r_o, r_d = gemm.forward_route(t, s.wo), gemm.forward_route(t, s.wd)
+    r_gu = gemm.forward_route(t, s.wgu) if s.pair is None else (gemm.PAIR_NT, s.pair[0])
+    routes, sizes = zip(r_o, r_gu, r_d)
+    gate, *up = _gate_up(s)
     *tail, y, normed = _lib.native().tail_forward(
-        residual, att, s.wo.w, s.wgu.w, s.wd.w, gain_post, gain_next, slot_gu, slot_d, slot_next, s.eps_post, s.eps_next,
-        *routes, gemm.TAIL_PARTS, gemm.workspace_for(residual.device, *sizes))
+        residual, att, s.wo.w, gate, s.wd.w, gain_post, gain_next, slot_gu, slot_d, slot_next, s.eps_post, s.eps_next,
+        *routes, gemm.TAIL_PARTS, gemm.workspace_for(residual.device, *sizes), *(up or (None,)))
     return y, normed, (*tail, y)
 
 
@@ -145,11 +154,16 @@ def _tail_backward(s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads
     dev = y.device
     nxt = _GainSum(grads_next, needs[1] and dn is not None, t, h, dev)
     post = _GainSum(grads_post, needs[0], t, h, dev)
-    routes, sizes, right = zip(*(gemm.backward_route(t, w) for w in (s.wo, s.wgu, s.wd)))
+    if s.pair is None:
+        r_gu, up = gemm.backward_route(t, s.wgu), None
+    else:
+        gate, up = s.wgu.pieces
+        r_gu = gemm.PAIR_NN, s.pair[1], gate
+    routes, sizes, right = zip(gemm.backward_route(t, s.wo), r_gu, gemm.backward_route(t, s.wd))
     dm, dgu, da, datt = _lib.native().tail_backward(
         dy, dn, mid, stats, gu, y, gain_post, gain_next, *right, s.wd.dy_slot(slot_d, t), s.wgu.dy_slot(slot_gu, t),
         s.wo.dy_slot(slot_o, t), post.scratch, post.acc, nxt.scratch, nxt.acc, *routes, gemm.TAIL_PARTS,
-        gemm.workspace_for(dev, *sizes))
+        gemm.workspace_for(dev, *sizes), up)
     tok_d, tok_gu, tok_o = s.wd.defer(slot_d, dm, act), s.wgu.defer(slot_gu, dgu, z), s.wo.defer(slot_o, da, att)
     return da, datt, post.result(), nxt.result(), tok_o, tok_gu, tok_d
 
@@ -225,7 +239,7 @@ class NormedLayer:
     layer's does its own input norm and projects all three from it (``wqkv`` in the place of ``wq``)."""
 
     __slots__ = ("wq", "wkv", "wo", "wgu", "wd", "eps_in", "eps_q", "eps_k", "eps_post", "eps_next", "hq", "hkv", "d",
-                 "scaling", "q_pos", "kv_pos", "inv_freq", "mask", "slots", "grad_slot")
+                 "scaling", "q_pos", "kv_pos", "inv_freq", "mask", "slots", "grad_slot", "pair")
 
     def __init__(self, wq, wkv, wo, wgu, wd, eps, heads, scaling, q_pos, kv_pos, inv_freq, mask):
         self.wq, self.wkv, self.wo, self.wgu, self.wd = wq, wkv, wo, wgu, wd
@@ -237,7 +251,7 @@ class NormedLayer:
     def constants(self, nq: int, nk: int):
         """See ``LayerStep.constants``; the mask's bounds for ``nq`` query rows and ``nk`` keys come first."""
         lo, hi, block_lo, block_hi, _, _ = A.mask_arguments(self.mask, nq, nk)
-        weights = (w.w for w in (self.wq, self.wkv, self.wo, self.wgu, self.wd) if w is not None)
+        weights = (*(w.w for w in (self.wq, self.wkv, self.wo, self.wd) if w is not None), *_gate_up(self))
         return (lo, hi, block_lo, block_hi, self.q_pos, self.kv_pos, self.inv_freq, *weights)
 
     @staticmethod

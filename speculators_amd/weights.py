@@ -116,6 +116,17 @@ def _cat_bf16(params) -> torch.Tensor:
     return out
 
 
+def _pair_as_it_lies(params) -> bool:
+    """Whether products may read two parameters as the halves of one weight: bf16 matrices of one shape, whole and aligned, on one
+    device."""
+    if len(params) != 2:
+        return False
+    a, b = params
+    return (a.dtype == b.dtype == torch.bfloat16 and a.dim() == 2 and a.shape == b.shape and a.shape[0] % 256 == 0
+            and a.shape[1] % 64 == 0 and a.device == b.device and a.is_contiguous() and b.is_contiguous()
+            and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0 and a.is_cuda)
+
+
 def _as_it_lies(p: torch.Tensor) -> torch.Tensor:
     """A bf16 parameter used alone: itself -- or a copy in rows of aligned chunks where it is a matrix stored otherwise
     (column by column, at an odd address, with an odd or overlapping row stride): the GEMM kernels take none of these."""
@@ -318,14 +329,14 @@ class _Uses:
 
 
 class Staged:
-    """One compute weight of this forward.  ``w``: bf16 ``[rows, cols]`` (or 1-D for a norm gain);
-    ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward
+    """One compute weight of this forward.  ``w``: bf16 ``[rows, cols]`` (or 1-D for a norm gain); where products may read its two
+    bf16 parameters as they lie (``pieces``, ``gemm.pair_routes``) it is put together when it is first asked for.  ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward
     is expected to run against it (the size of the input / output-gradient buffers)."""
 
-    __slots__ = ("w", "token", "rows_of", "_wt", "records", "x_slot", "take", "dy_slot", "defer", "mark", "grad_buffer")
+    __slots__ = ("_w", "pieces", "token", "rows_of", "_wt", "records", "x_slot", "take", "dy_slot", "defer", "mark", "grad_buffer")
 
     def __init__(self, w, rows_of, uses: int = 1, bf16_params: bool = False):
-        self.w = w
+        self._w, self.pieces = w if isinstance(w, tuple) else (w, None)
         self.token = None  # fp32 stand-in of w's shape that carries the gradient edge (trainable only)
         self.rows_of = rows_of
         self._wt = None
@@ -335,9 +346,16 @@ class Staged:
 
     def train(self, w, token):
         """The compute weight and its token, as the staging node made them."""
-        self.w, self.token = w, token
+        self._w, self.pieces = w if isinstance(w, tuple) else (w, None)
+        self.token = token
         r = self.records
-        r.shape, r.device, r.trainable = w.shape, w.device, True
+        r.shape, r.device, r.trainable = token.shape, token.device, True
+
+    @property
+    def w(self) -> torch.Tensor:
+        if self._w is None:
+            self._w = _cat_bf16(self.pieces)
+        return self._w
 
     @property
     def trainable(self) -> bool:
@@ -419,10 +437,13 @@ class _StageAll(torch.autograd.Function):
             group = params[at:at + n]
             at += n
             w = made.get(i)
+            if w is None and _pair_as_it_lies(group):
+                out += [None, _lib.zero(group[0].device).expand(2 * group[0].shape[0], group[0].shape[1])]
+                continue
             if w is None:
                 w = _as_it_lies(group[0]) if n == 1 and group[0].dtype == torch.bfloat16 else _cat_bf16(group)
             out += [w, _lib.zero(w.device).expand(w.shape)]
-        ctx.mark_non_differentiable(*out[::2])
+        ctx.mark_non_differentiable(*(w for w in out[::2] if w is not None))
         return tuple(out)
 
     @staticmethod
@@ -534,7 +555,7 @@ class WeightStager:
         staged = [Staged(None, [p.shape[0] for p in g], self._uses, all(p.dtype == torch.bfloat16 for p in g)) for g in groups]
         out = _StageAll.apply([st.records for st in staged], dict(enumerate(made or ())), [len(g) for g in groups], *(p for g in groups for p in g))
         for st, g, w, token in zip(staged, groups, out[::2], out[1::2], strict=True):
-            st.train(w, token)
+            st.train((None, tuple(p.detach() for p in g)) if w is None else w, token)
             self._fwd[tuple(id(p) for p in g)] = st
 
     def get(self, *params) -> Staged:
@@ -552,9 +573,12 @@ class WeightStager:
             fkey = tuple((p.data_ptr(), p._version, p.dtype) for p in params)
             kept = self._frozen.get(key)
             if kept is None or kept[0] != fkey:
-                w = _as_it_lies(params[0]) if len(params) == 1 and params[0].dtype == torch.bfloat16 \
-                    else _cat_bf16(params)
-                kept = (fkey, Staged(w, rows_of))
+                if any(p.requires_grad for p in params) and _pair_as_it_lies(params):
+                    w = None, tuple(p.detach() for p in params)
+                else:
+                    w = _as_it_lies(params[0]) if len(params) == 1 and params[0].dtype == torch.bfloat16 \
+                        else _cat_bf16(params)
+                kept = (fkey, Staged(w, rows_of, self._uses))
                 if not any(p.requires_grad for p in params):
                     self._frozen[key] = kept  # trainable weights seen under no_grad are not kept
             st = kept[1]
