@@ -471,6 +471,11 @@ def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
 
 
 @functools.lru_cache(maxsize=4096)
+def _lines_matter(mode: str, m: int, n: int, k: int) -> bool:
+    return mode == "mixed" and not _own_forward(m, n, k) and _walking_forward(m, n, k)
+
+
+@functools.lru_cache(maxsize=4096)
 def _forward_route(mode: str, parts: int, m: int, n: int, k: int, lines: bool = True):
     """``(route, workspace elements)`` of ``_project`` for contiguous rows (``lines``: of a weight of ``_rows_in_lines``)."""
     if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k) and not (lines and _walking_forward(m, n, k))):
@@ -485,7 +490,11 @@ def _forward_route(mode: str, parts: int, m: int, n: int, k: int, lines: bool = 
 
 
 def forward_route(m: int, staged):
-    return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *staged.w.shape, _rows_in_lines(staged.w))
+    w = staged.w
+    route = _forward_route(DECODER_GEMM, TAIL_PARTS, m, *w.shape)
+    if _lines_matter(DECODER_GEMM, m, *w.shape) and not _rows_in_lines(w):
+        return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *w.shape, False)
+    return route
 
 
 @functools.lru_cache(maxsize=4096)
