@@ -191,8 +191,11 @@ class DecoderLayer(nn.Module):
                 or not cache.get("steps") or (self.first and cfg.norm_before_residual)):
             return None
         mlp = self.mlp
-        ws = self._stager.get_all((att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), (att.o_proj.weight,),
-                                  (mlp.gate_proj.weight, mlp.up_proj.weight), (mlp.down_proj.weight,))
+        ws = cache.get("weights")
+        if ws is None:  # (the layer's cache is one forward's, as what the stager hands out)
+            ws = cache["weights"] = self._stager.get_all(
+                (att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), (att.o_proj.weight,),
+                (mlp.gate_proj.weight, mlp.up_proj.weight), (mlp.down_proj.weight,))
         if torch.is_grad_enabled() and not all(w.trainable for w in ws):
             return None
         kvc = cache.get("kv")
