@@ -330,8 +330,9 @@ class _Uses:
 
 class Staged:
     """One compute weight of this forward.  ``w``: bf16 ``[rows, cols]`` (or 1-D for a norm gain); where products may read its two
-    bf16 parameters as they lie (``pieces``, ``gemm.pair_routes``) it is put together when it is first asked for.  ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward
-    is expected to run against it (the size of the input / output-gradient buffers)."""
+    bf16 parameters as they lie (``pieces``, ``gemm.pair_routes``) it is put together when it is first asked for.
+    ``rows_of``: the row count of every parameter in it; ``uses``: how many products the forward is expected to run against
+    it (the size of the input / output-gradient buffers)."""
 
     __slots__ = ("_w", "pieces", "token", "rows_of", "_wt", "records", "x_slot", "take", "dy_slot", "defer", "mark", "grad_buffer")
 
@@ -553,7 +554,8 @@ class WeightStager:
         for g in groups:
             _check_params(g)
         staged = [Staged(None, [p.shape[0] for p in g], self._uses, all(p.dtype == torch.bfloat16 for p in g)) for g in groups]
-        out = _StageAll.apply([st.records for st in staged], dict(enumerate(made or ())), [len(g) for g in groups], *(p for g in groups for p in g))
+        out = _StageAll.apply([st.records for st in staged], dict(enumerate(made or ())), [len(g) for g in groups],
+                              *(p for g in groups for p in g))
         for st, g, w, token in zip(staged, groups, out[::2], out[1::2], strict=True):
             st.train((None, tuple(p.detach() for p in g)) if w is None else w, token)
             self._fwd[tuple(id(p) for p in g)] = st
