@@ -122,6 +122,7 @@ PyMethodDef g_methods[] = {
 #include "binding_list.h"
     SPX_HOST("attention", spx_node_attention)
     SPX_HOST("row_loss", spx_node_row_loss)
+    SPX_HOST("wanted", spx_node_wanted)
     SPX_HOST("product", spx_layer_product)
     SPX_HOST("tail_forward", spx_layer_tail_forward)
     SPX_HOST("tail_backward", spx_layer_tail_backward)

@@ -4,6 +4,7 @@
 // 1024 tokens of the 1B attention shape, forward and backward issued: 150 -> 75 us; a loss function 130 -> 75 us.
 
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_function.h>
 
 #include "host_common.h"
 
@@ -182,5 +183,19 @@ PyObject* spx_node_row_loss(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor out = RowLoss::apply(x, y, op);
   released.lock();
   return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// (ctx.needs_input_grad of a Python node says what requires a gradient, not what this pass was asked for)
+PyObject* spx_node_wanted(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 1 && THPFunction_Check(args[0]), "wanted takes the context of an autograd function");
+  const auto node = reinterpret_cast<THPFunction*>(args[0])->cdata.lock();
+  TORCH_CHECK_VALUE(node, "the context belongs to no node of a graph");
+  const Py_ssize_t inputs = (Py_ssize_t)node->num_outputs();
+  PyObject* const all = PyTuple_New(inputs);
+  if (!all) return nullptr;
+  for (Py_ssize_t i = 0; i < inputs; ++i) PyTuple_SET_ITEM(all, i, PyBool_FromLong(node->task_should_compute_output(i)));
+  return all;
   END_HANDLE_TH_ERRORS
 }

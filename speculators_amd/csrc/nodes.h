@@ -8,6 +8,9 @@ PyObject* spx_node_attention(PyObject*, PyObject* const* args, Py_ssize_t n);
 // row_loss(op, logits [..., V], targets) -> float32 [...]
 PyObject* spx_node_row_loss(PyObject*, PyObject* const* args, Py_ssize_t n);
 
+// wanted(ctx of a Python node) -> for each of the tensors it was applied to, whether the running backward pass asks for its gradient
+PyObject* spx_node_wanted(PyObject*, PyObject* const* args, Py_ssize_t n);
+
 // The launches of a decoder layer in sequence (layer_host.cpp), called by layer.py; arguments positional, as read there.
 PyObject* spx_layer_product(PyObject*, PyObject* const* args, Py_ssize_t n);
 PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n);

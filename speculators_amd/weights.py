@@ -220,13 +220,17 @@ class _Uses:
         return -1
 
     # ---- backward side
+    def drop(self):
+        """Forgets what the uses recorded."""
+        self._dys, self._live, self._extras, self._marked, self._acc = None, [], [], False, None
+
     def _enter_pass(self):
         """What the uses record belongs to ONE backward pass, which ends in ``finish`` when autograd
         reaches the staging node.  A pass that never got there (``autograd.grad`` for other inputs
         over a retained graph) must not leak its records into the next one."""
         task = torch._C._current_graph_task_id()
         if task != self._task:
-            self._dys, self._live, self._extras, self._marked, self._acc = None, [], [], False, None
+            self.drop()
             self._task = task
 
     def dy_slot(self, r0: int, rows: int):
@@ -290,7 +294,7 @@ class _Uses:
             pair = self._dys[rows], self._xs[rows]
         if not (_tn_ok(pair[0]) and _tn_ok(pair[1])):
             return None
-        self._dys, self._live, self._extras, self._marked = None, [], [], False
+        self.drop()
         return pair
 
     def finish(self, bf16_ok: bool = False):
@@ -324,7 +328,7 @@ class _Uses:
             acc = wgrad_product(self._dys[r0:r0 + n], self._xs[r0:r0 + n], acc)
         for dy2, x2 in self._extras:
             acc = wgrad_product(dy2, x2, acc)
-        self._dys, self._live, self._extras, self._marked, self._acc = None, [], [], False, None
+        self.drop()
         return acc
 
 
@@ -451,7 +455,8 @@ class _StageAll(torch.autograd.Function):
     def backward(ctx, *gs):
         from .gemm import gemm_tn_all
 
-        needed = ctx.needs_input_grad[3:]
+        # (a node a weight ran where its own weight was asked for: this one is reached where any of the layer's is)
+        needed = _lib.native().wanted(ctx)
         groups, at = [], 0
         for n in ctx.sizes:
             groups.append(slice(at, at + n))
@@ -460,6 +465,7 @@ class _StageAll(torch.autograd.Function):
         for i, (uses, group) in enumerate(zip(ctx.records, groups, strict=True)):
             g = gs[2 * i + 1]
             if not any(needed[group]):
+                uses.drop()
                 continue
             bf16 = all(dt == torch.bfloat16 for dt in ctx.dtypes[group])
             pair = uses.sole()
