@@ -282,6 +282,7 @@ class _Uses:
 
     def sole(self):
         """``(dy, x)`` where one product is all there is to the weight gradient (the records are dropped then), else None."""
+        self._enter_pass()  # (the node may be reached by other weights' uses alone)
         if self._acc is not None or len(self._extras) > 1 or bool(self._extras) == bool(self._live):
             return None
         if self._extras:
@@ -302,6 +303,7 @@ class _Uses:
         per run of adjacent uses in the buffers -- normally one -- plus one per outside use.
         ``bf16_ok``: the parameters are bf16, so when ONE product is all there is, it writes bf16
         itself (the same fp32 accumulation and the same one rounding as a cast of its fp32 result)."""
+        self._enter_pass()
         acc = self._acc
         runs: list = []
         for r0, n in sorted(self._live):

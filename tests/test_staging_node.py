@@ -89,3 +89,43 @@ def test_wanted_takes_contexts_alone():
     for wrong in (torch.ones(2), None, object()):
         with pytest.raises(TypeError, match="context"):
             _lib.native().wanted(wrong)
+
+
+class _Product(torch.autograd.Function):
+    """``x @ w.T`` that leaves its weight gradient to the staging node, as ``gemm._StagedLinear``."""
+
+    @staticmethod
+    def forward(ctx, x, w, _token, records):
+        ctx.save_for_backward(x, w)
+        ctx.records = records
+        return x @ w.T
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        return dy @ w, None, ctx.records.defer(-1, dy, x), None
+
+
+def _two_products(monkeypatch):
+    monkeypatch.setattr(weights, "wgrad_product", lambda dy, x, acc: dy.T @ x if acc is None else acc + dy.T @ x)
+    a, b = (torch.nn.Parameter(torch.randn(6, 8)) for _ in range(2))
+    records = [weights._Uses(1, False) for _ in range(2)]
+    out = weights._StageAll.apply(records, {i: w.detach() for i, w in enumerate((a, b))}, [1, 1], a, b)
+    for r, token in zip(records, out[1::2], strict=True):
+        r.shape, r.device, r.trainable = token.shape, token.device, True
+    x = torch.randn(5, 8, requires_grad=True)
+    return a, b, x, [_Product.apply(x, out[2 * i], out[2 * i + 1], records[i]).square().sum() for i in range(2)]
+
+
+def test_records_of_an_earlier_pass_are_not_used(monkeypatch):
+    """A pass for the input alone leaves what the uses recorded; the next one, which reaches the node by one of the two, forms that
+    one's gradient and no other."""
+    a, b, x, (loss_a, loss_b) = _two_products(monkeypatch)
+    torch.autograd.grad(loss_a + loss_b, (x,), retain_graph=True)
+    loss_a.backward(retain_graph=True)
+    assert b.grad is None
+    torch.testing.assert_close(a.grad, 2 * (x @ a.T).T @ x)
+    a.grad = None
+    (loss_a + loss_b).backward()
+    for p in (a, b):
+        torch.testing.assert_close(p.grad, 2 * (x @ p.T).T @ x)
