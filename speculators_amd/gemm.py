@@ -259,10 +259,10 @@ class _TnProduct(ctypes.Structure):  # spx_tn_product
 
 @functools.lru_cache(maxsize=4096)
 def _tn_list_plan(shapes: tuple, fp32: bool):
-    """``(predicted us, workspace elements)`` of ``spx_gemm_bf16_tn_list`` over products ``(T, M, N, lda, ldb)``; us is
+    """``(predicted us, workspace elements)`` of ``spx_gemm_bf16_tn_list`` over products ``(T, M, N, lda, ldb, ldc)``; us is
     negative where it does not take them."""
     lib = _lib.load()
-    items = (_TnProduct * len(shapes))(*(_TnProduct(0, lda, 0, ldb, 0, n, m, n, t) for t, m, n, lda, ldb in shapes))
+    items = (_TnProduct * len(shapes))(*(_TnProduct(0, lda, 0, ldb, 0, ldc, m, n, t) for t, m, n, lda, ldb, ldc in shapes))
     return (lib.spx_gemm_tn_list_us(items, len(shapes), int(fp32)),
             lib.spx_gemm_tn_list_workspace_bytes(items, len(shapes), int(fp32)) // 4)
 
@@ -277,18 +277,22 @@ def _tn_alone(shape: tuple, fp32: bool):
     return (walks, True) if 0 < walks < us or (walks > 0 and lib.spx_gemm_tn_tile(m, n, t) == 0) else (us, False)
 
 
+def _tn_shape(a, b, out) -> tuple:
+    n = b.shape[1]
+    return a.shape[0], a.shape[1], n, a.stride(0), b.stride(0), n if out is None else out.stride(0)
+
+
 def _walks(shape: tuple, fp32: bool) -> bool:
     return _tn_alone(shape, fp32)[1]
 
 
 def _whole_lines(a, b, out) -> bool:
     return (a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0 and a.shape[1] % 8 == 0 and b.shape[1] % 8 == 0
-            and a.stride(0) % 8 == 0 and b.stride(0) % 8 == 0
-            and (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)))
+            and a.stride(0) % 8 == 0 and b.stride(0) % 8 == 0 and (out is None or out.data_ptr() % 16 == 0))
 
 
 def _tn_list(pairs, fp32: bool, outs):
-    ws_numel = _tn_list_plan(tuple((a.shape[0], a.shape[1], b.shape[1], a.stride(0), b.stride(0)) for a, b in pairs), fp32)[1]
+    ws_numel = _tn_list_plan(tuple(_tn_shape(a, b, out) for (a, b), out in zip(pairs, outs, strict=True)), fp32)[1]
     ws = _split_workspace(pairs[0][0].device, ws_numel) if ws_numel else None
     return _lib.native().products_tn(fp32, ws, *(x for (a, b), out in zip(pairs, outs, strict=True) for x in (a, b, out)))
 
@@ -297,7 +301,7 @@ def gemm_tn_all(pairs, out_dtype: torch.dtype):
     """``gemm_tn`` of every ``(a, b)``: in one launch where the walking kernel takes them all and is predicted to be faster than
     each alone (the layer of the 1B shape over 1536 rows: 219 us in four launches, 167 in one)."""
     fp32 = out_dtype == torch.float32
-    shapes = tuple((a.shape[0], a.shape[1], b.shape[1], a.stride(0), b.stride(0)) for a, b in pairs)
+    shapes = tuple(_tn_shape(a, b, None) for a, b in pairs)
     if 1 < len(pairs) <= 8 and all(s[0] > 0 for s in shapes) and all(_whole_lines(a, b, None) for a, b in pairs):
         us = _tn_list_plan(shapes, fp32)[0]
         if 0 < us < sum(_tn_alone(s, fp32)[0] for s in shapes):
@@ -328,7 +332,7 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None,
     elif out.shape != (m, n) or out.dtype not in (torch.bfloat16, torch.float32) or out.stride(1) != 1:
         raise ValueError(f"out must be a bf16 or fp32 [{m}, {n}] tensor with unit column stride")
     fp32 = (out_dtype if out is None else out.dtype) == torch.float32
-    if not accumulate and t > 0 and _walks((t, m, n, a.stride(0), b.stride(0)), fp32) and _whole_lines(a, b, out):
+    if not accumulate and t > 0 and _walks(_tn_shape(a, b, out), fp32) and _whole_lines(a, b, out):
         return _tn_list([(a, b)], fp32, [out])[0]
     # 32-bit byte offsets inside the kernel: a contraction that spans 2 GiB or more of an
     # operand is fed in bands of rows, every band after the first added to the result.  A bf16 result of several

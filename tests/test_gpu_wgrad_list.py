@@ -45,8 +45,24 @@ def test_list_against_float64(name, fp32, pad):
 def test_the_plan_cuts_where_the_tests_say_so():
     from speculators_amd.gemm import _tn_list_plan
 
-    cut = {name: _tn_list_plan(tuple((*s, s[1], s[2]) for s in shapes), True)[1] > 0 for name, shapes in LISTS.items()}
+    cut = {name: _tn_list_plan(tuple((*s, s[1], s[2], s[2]) for s in shapes), True)[1] > 0 for name, shapes in LISTS.items()}
     assert [name for name, is_cut in cut.items() if is_cut] == [name for name in LISTS if "in parts" in name]
+
+
+@pytest.mark.parametrize("dtype,stride", [(torch.float32, 65544), (torch.float32, 1 << 21), (torch.bfloat16, 1 << 22)])
+def test_results_in_rows_far_apart(dtype, stride):
+    """A tile's 256 rows of the result span 2 GiB: not on the walking kernel, which offsets them in 32 bits, but as before it."""
+    from speculators_amd.gemm import _tn_shape, _walks, gemm_tn
+
+    (a, b), = _operands([(300, 8, 65528)], 256)
+    out = torch.full((8 * stride,), 3.0, device="cuda", dtype=dtype).view(8, stride)[:, :65528]
+    fp32 = dtype == torch.float32
+    assert _walks(_tn_shape(a, b, None), fp32) and _walks(_tn_shape(a, b, out), fp32) == (stride == 65544)
+    assert gemm_tn(a, b, out) is out
+    want = a.double().t() @ b.double()
+    tol = (2e-6 * 300 ** 0.5 if fp32 else 2 ** -8) * want.abs().max().item() + 1e-4
+    assert (out.double() - want).abs().max().item() <= tol
+    assert (torch.as_strided(out, (8, stride - 65528), (stride, 1), 65528) == 3).all()
 
 
 def test_rules():
