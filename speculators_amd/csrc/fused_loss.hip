@@ -1392,7 +1392,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     for (int i = 0; i < 8; ++i) z += fast_exp2(fmaf(x[i], kLog2e, -m));
   };
 
-  float top = 0.f;  // the target row's largest
+  float top = 0.f;  // the target row's largest, see below
   float lt2 = 0.f;  // base-2 log-sum-exp of the target row
   int label;
   if (a.targets) {
@@ -1410,7 +1410,8 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     }
     reduce(best, label, z, none, kY);
     lt2 = z;
-    top = best;
+    // (within 2^119: from a larger one the difference to the type's lowest value would overflow, and times p = 0 be NaN)
+    top = fminf(fmaxf(best, -0x1p119f), 0x1p119f);
     if (kY) {
       float sum = 0.f;
 #pragma unroll

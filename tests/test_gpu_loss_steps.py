@@ -181,3 +181,25 @@ def test_target_rows_held_as_probabilities(vocab, name):
     mask[0, 25] = 1
     want, got = _one_by_one(x, w, y, mask, 0.9, config), _together(x, w, y, mask, 0.9, config)
     assert torch.equal(got[0].isnan(), want[0].isnan())
+
+
+@pytest.mark.parametrize("top", [2.0 ** 100, 2.0 ** 121, 2.0 ** 125, 1.5 * 2.0 ** 121])
+@pytest.mark.parametrize("name", ["kl_div", '{"tv": 1.5, "kl_div": 0.25, "ce": 0.125}'])
+def test_a_target_row_at_the_edges_of_the_type(top, name):
+    """A largest logit beyond 1.3e36 beside the lowest value.  A power of two times log2(e) is exact, and so are the log-sum-exp and
+    the probability of one: the loss is finite as step by step.  Others round to probabilities of zero: no NaN from these."""
+    from speculators_amd import losses as L
+
+    config = L.resolve_loss_config(name)
+    x, w, y, mask = _case(20, 2, 4104, 6)
+    y[0, 11], mask[0, 11] = torch.finfo(torch.bfloat16).min, 1
+    y[0, 11, 40] = top
+    want, got = _one_by_one(x, w, y, mask, 0.9, config), _together(x, w, y, mask, 0.9, config)
+    assert not got[0].isnan()
+    if top == 1.5 * 2.0 ** 121:
+        return
+    assert got[0].isfinite() and want[0].isfinite()
+    # sums of terms of the size of top, each rounded to 24 bits, and the log-sum-exp of that size
+    assert (got[0] - want[0]).abs() <= 16 * 2.0 ** -24 * abs(top)
+    for a, b in zip(got[4], want[4], strict=True):
+        _close(a, b, 2.0 ** -8)
