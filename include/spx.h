@@ -762,7 +762,8 @@ int spx_gemm_bf16_auto_parts(int form, const void* a, int64_t lda, const void* b
 /* spx_gemm_bf16_auto with the rows of b in two matrices of as many rows (N / 2 each, form 1: K / 2), ldb apart in both: the weights
  * of two projections of one input as they lie.  For sizes that spx_gemm_pair_takes accepts (256 x 256 tiles by workgroups that
  * walk them, N / 2 a multiple of 256, form 1: K / 2 of 64); another size is refused.  c's rows are 16-byte aligned.  Workspace and
- * parts (form 1; NULL: they are added) as for spx_gemm_bf16_auto and spx_gemm_bf16_auto_parts. */
+ * parts (form 1; NULL: they are added) as for spx_gemm_bf16_auto and spx_gemm_bf16_auto_parts, the workspace not NULL where form 1
+ * asks for one. */
 int spx_gemm_pair_takes(int form, int64_t M, int64_t N, int64_t K, int64_t ldb, int32_t max_parts);
 int spx_gemm_bf16_pair(int form, const void* a, int64_t lda, const void* b, const void* b2, int64_t ldb, void* c, int64_t ldc,
                        int64_t M, int64_t N, int64_t K, int32_t max_parts, void* workspace, int64_t workspace_bytes,

@@ -555,8 +555,9 @@ static int auto_product(const char* fname, int form, const void* a, int64_t lda,
     const WalkArgs w = {p.A, lda, p.B, ldb, reinterpret_cast<uint16_t*>(c), ldc, M, N, K, m_live, p.part_ws, 1, 0, tile::kCus,
                         wgs, RowGrade{}, ch.parts, reinterpret_cast<const uint16_t*>(b2)};
     if (int rc = walk(fname, true, w, st)) return rc;
-  } else if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st)) {
-    return rc;
+  } else {
+    SPX_REQ_FN(!b2, "a second half of b: sizes that workgroups walk");
+    if (int rc = form ? tile::launch_dense<true>(fname, ch.tile, p, st) : tile::launch_dense<false>(fname, ch.tile, p, st)) return rc;
   }
   if (ch.parts == 1) return SPX_OK;
   if (left) {
@@ -606,7 +607,9 @@ extern "C" int spx_gemm_bf16_pair(int form, const void* a, int64_t lda, const vo
   SPX_REQ_FN(ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0, "ldc must be a multiple of 8 and c 16-byte aligned");
   SPX_REQ_FN(spx_gemm_pair_takes(form, M, N, K, ldb, max_parts) && 256 * ldc * 2 < 0x7ffffff0ll, "sizes that spx_gemm_pair_takes refuses");
   if (form) {
-    SPX_REQ_FN(workspace_bytes >= spx_gemm_auto_workspace_bytes(1, M, N, K, max_parts), "workspace too small");
+    const int64_t need = spx_gemm_auto_workspace_bytes(1, M, N, K, max_parts);
+    SPX_REQ_FN(need == 0 || (workspace && ((uintptr_t)workspace) % 16 == 0 && workspace_bytes >= need),
+               "workspace too small, null or unaligned");
     return auto_product(fname, 1, a, lda, b, ldb, c, ldc, M, N, K, nullptr, max_parts, workspace, workspace_bytes, parts, stream, b2);
   }
   const bool cut = max_parts > 1 && workspace && ((uintptr_t)workspace) % 16 == 0 && workspace_bytes >= spx_gemm_tail_workspace_bytes();

@@ -152,3 +152,15 @@ def test_product_workspaces_belong_to_one_thread():
     thread.join()
     assert other[0][0] and other[0][1]() is None
     assert gemm._split_workspace(cpu, 64) is mine
+
+
+@pytest.mark.parametrize("workspace,room", [(None, 1 << 30), (4100, 1 << 30), (4096, 1 << 20)])
+def test_a_pair_product_cut_whole_needs_its_workspace(workspace, room):
+    """Without one its size has another choice, whose kernels know no second half of the weight: refused before any launch."""
+    from speculators_amd import _lib
+
+    lib = _lib.load()
+    m, n, k = 888, 2048, 16384
+    assert lib.spx_gemm_pair_takes(1, m, n, k, n, 4) and lib.spx_gemm_auto_workspace_bytes(1, m, n, k, 4) > 1 << 20
+    rc = lib.spx_gemm_bf16_pair(1, 4096, k, 4096, 4096, n, 4096, n, m, n, k, 4, workspace, room, None, None)
+    assert rc == 1 and b"workspace" in lib.spx_last_error()
