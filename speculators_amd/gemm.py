@@ -405,7 +405,7 @@ def _on_192_rows(m: int, n: int, k: int, parts: int) -> bool:
     return tile in (4, 5) and m <= 1024 and k <= 3072
 
 
-def _own_forward(m: int, n: int, k: int) -> bool:
+def _own_forward(m: int, n: int, k: int, parts: int | None = None) -> bool:
     """Whether the forward product of a decoder projection runs on this library's kernels in "mixed" (ratios: own time to
     hipBLASLt's).
 
@@ -420,19 +420,19 @@ def _own_forward(m: int, n: int, k: int) -> bool:
     products (0.83), from 4096 on 0.80 - 1.33 over 41 (1.06; 8B gate/up at 260 - 960 rows 0.99 - 1.11, 70B q/k/v at 777 - 1024
     1.24 - 1.33, 70B gate/up 1.02 - 1.21).
     (profiles/decoder_forward_products.txt.)"""
-    big, ws_numel, _ = _plan(2, m, n, k, TAIL_PARTS)  # (the choice without them is that of a device row count)
+    parts = TAIL_PARTS if parts is None else parts
+    big, ws_numel, _ = _plan(2, m, n, k, parts)  # (the choice without them is that of a device row count)
     if not big:
         if ws_numel > 0 or m <= 1024 or m * n <= 256 * 256 * 128:
             return True
     else:
         tiles = -(-m // 256) * -(-n // 256)
-        if TAIL_PARTS > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS:
+        if parts > 1 and 0 < tiles % _CUS <= _CUS // 2 and k >= 64 * 16 * 2 and tiles < 2 * _CUS:
             return True
-    return _on_192_rows(m, n, k, TAIL_PARTS)
+    return _on_192_rows(m, n, k, parts)
 
 
-@functools.lru_cache(maxsize=4096)
-def _walking_forward(m: int, n: int, k: int) -> bool:
+def _walking_forward(m: int, n: int, k: int, parts: int | None = None) -> bool:
     """Of what ``_own_forward`` leaves to the library, the products that workgroups which walk the large tiles take as fast or
     faster (ratios: own time to hipBLASLt's, 156 products of 700 to 32760 rows of the 1B, 8B and 70B shapes and others; each is a
     library call of some 25 us on the host less, too).
@@ -442,11 +442,16 @@ def _walking_forward(m: int, n: int, k: int) -> bool:
     1.01, 70B gate/up 0.90 - 0.93).  Contractions from 16384 on: 0.64 - 1.02 over 22 (0.86).  Left to the library: whole
     rounds over 4096 to 16383, 0.84 - 1.05 over 55 (1.00, but 1.01 - 1.05 where N is a power of two or three of them), and
     the tiles of 192 rows."""
-    if not m or k % 64 or n % 8 or _lib.load().spx_gemm_auto_tile(0, m, n, k, TAIL_PARTS):
+    return _walks_as_fast(m, n, k, TAIL_PARTS if parts is None else parts)
+
+
+@functools.lru_cache(maxsize=4096)
+def _walks_as_fast(m: int, n: int, k: int, parts: int) -> bool:
+    if not m or k % 64 or n % 8 or _lib.load().spx_gemm_auto_tile(0, m, n, k, parts):
         return False
     if k < 4096:
         return True
-    return m > 1024 and (k >= 16384 or _forward_route("spx", TAIL_PARTS, m, n, k)[0] == TAIL)
+    return m > 1024 and (k >= 16384 or _forward_route("spx", parts, m, n, k)[0] == TAIL)
 
 
 def _rows_in_lines(t: torch.Tensor) -> bool:
@@ -475,14 +480,15 @@ def _project_back(dy2: torch.Tensor, staged) -> torch.Tensor:
 
 
 @functools.lru_cache(maxsize=4096)
-def _lines_matter(mode: str, m: int, n: int, k: int) -> bool:
-    return mode == "mixed" and not _own_forward(m, n, k) and _walking_forward(m, n, k)
+def _lines_matter(mode: str, parts: int, m: int, n: int, k: int) -> bool:
+    return mode == "mixed" and not _own_forward(m, n, k, parts) and _walking_forward(m, n, k, parts)
 
 
 @functools.lru_cache(maxsize=4096)
 def _forward_route(mode: str, parts: int, m: int, n: int, k: int, lines: bool = True):
     """``(route, workspace elements)`` of ``_project`` for contiguous rows (``lines``: of a weight of ``_rows_in_lines``)."""
-    if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k) and not (lines and _walking_forward(m, n, k))):
+    if mode == "hipblaslt" or (mode == "mixed" and not _own_forward(m, n, k, parts)
+                               and not (lines and _walking_forward(m, n, k, parts))):
         return LINEAR, 0
     big, ws_numel, _ = _plan(0, m, n, k, parts)
     if not big and k % 8 == 0:
@@ -496,7 +502,7 @@ def _forward_route(mode: str, parts: int, m: int, n: int, k: int, lines: bool = 
 def forward_route(m: int, staged):
     w = staged.w
     route = _forward_route(DECODER_GEMM, TAIL_PARTS, m, *w.shape)
-    if _lines_matter(DECODER_GEMM, m, *w.shape) and not _rows_in_lines(w):
+    if _lines_matter(DECODER_GEMM, TAIL_PARTS, m, *w.shape) and not _rows_in_lines(w):
         return _forward_route(DECODER_GEMM, TAIL_PARTS, m, *w.shape, False)
     return route
 

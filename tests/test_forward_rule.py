@@ -37,3 +37,28 @@ def test_products_that_workgroups_walk(rows, n, k, here):
     assert not gemm._own_forward(rows, n, k) and gemm._walking_forward(rows, n, k) == here
     assert (gemm._forward_route("mixed", gemm.TAIL_PARTS, rows, n, k)[0] != gemm.LINEAR) == here
     assert gemm._forward_route("mixed", gemm.TAIL_PARTS, rows, n, k, False)[0] == gemm.LINEAR
+
+
+def test_routes_go_by_the_parts_that_are_asked_for(monkeypatch):
+    """A route of another number of parts than the running one is the route that runs with that number, whatever was asked first."""
+    shapes = [(m, n, k) for m in (300, 1500, 3001, 4096, 5000) for n, k in ((28672, 4096), (6144, 16384), (6144, 8192), (4096, 4096))]
+
+    def forget():
+        for f in vars(gemm).values():
+            getattr(f, "cache_clear", lambda: None)()
+
+    def routes(parts):
+        return [gemm._forward_route("mixed", parts, *s, lines) for s in shapes for lines in (False, True)]
+
+    def walk():
+        return [gemm._walking_forward(*s) for s in shapes]
+
+    forget()
+    asked, walked = {p: routes(p) for p in (4, 1)}, {}
+    for parts in (1, 4):
+        monkeypatch.setattr(gemm, "TAIL_PARTS", parts)
+        walked[parts] = walk()
+        forget()
+        assert routes(parts) == asked[parts] and walk() == walked[parts]
+    assert asked[1] != asked[4] and walked[1] != walked[4]
+    forget()
