@@ -272,6 +272,13 @@ constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (kFifth)
                           {192, 256, 1, 0.76f, 0.35f, 5.1f},
                           {256, 256, 1, 0.78f, 0.47f, 7.4f},   // gemm_bf16_walk.hip
                           {192, 128, 1, 0.45f, 0.18f, 4.3f}};
+// kFifth of the second form where N is no multiple of 256: those workgroups do not walk (walk_takes), and the 256 x 256 tile by eight
+// waves takes 6 % longer than the price above.  5 % rms over 40 products of 512 .. 8192 rows -> 896 .. 5000 columns; chosen
+// with it / with the price above, us: 1400 x 8192 -> 4160 92.0 / 96.2, 700 x 11520 -> 2880 54.3 / 57.0, 8192 x 4096 -> 2880 167.0 /
+// 172.7, the other 37 alike: 1.009 of the best candidate in place of 1.013 in the geometric mean.  (Contractions that end
+// inside a slab do not walk either, but there all candidates take as much longer: 30 products a b and 36 a b^T
+// are within 1.02 of the best as they are priced.)
+constexpr Config kNNAside = {256, 256, 1, 0.96f, 0.30f, 7.6f};
 // Weight gradients (contraction slow in both operands): the candidates beside the 256 x 256 kernel of gemm_bf16_tn.hip,
 // which keeps whole rounds of its tiles and is given up only for a predicted tenth.  Fitted the same way to 128 products
 // (results of 1 .. 768 large tiles, 256 .. 20000 rows, up to 12 parts; 6 - 13 % rms).  Over them the choice takes 0.52 of that
@@ -323,7 +330,7 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
     if (cut) best.us += predict(c, cut * tp, (slabs + tp - 1) / tp) + reduce_us((float)(cut * tp * 65536));
   }
   for (int t = 1; t < (nn ? 7 : form == 2 ? (int)k192x256 : 6); ++t) {
-    const Config& c = table[t];
+    const Config& c = nn && t == kFifth && N % 256 ? kNNAside : table[t];
     const int64_t tiles = ((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn);
     const int64_t cap = (int64_t)kCus * c.per_cu;
     for (int parts = 1; parts <= kMaxParts; ++parts) {

@@ -62,3 +62,11 @@ def test_routes_go_by_the_parts_that_are_asked_for(monkeypatch):
         assert routes(parts) == asked[parts] and walk() == walked[parts]
     assert asked[1] != asked[4] and walked[1] != walked[4]
     forget()
+
+
+# (rows, columns, contraction, tile): results of no whole number of 256 columns, where the large tile is not the walking one, and
+# of such a number, where it is
+@pytest.mark.parametrize("m,n,k,tile", [(1400, 4160, 8192, 2), (8192, 2880, 4096, 2), (700, 2880, 11520, 4),
+                                        (1400, 2048, 16384, 5), (8192, 4096, 14336, 5), (3500, 2048, 16384, 5)])
+def test_input_gradients_on_large_tiles(m, n, k, tile):
+    assert _lib.load().spx_gemm_auto_tile(1, m, n, k, 4) == tile
