@@ -49,6 +49,25 @@ def test_the_plan_cuts_where_the_tests_say_so():
     assert [name for name, is_cut in cut.items() if is_cut] == [name for name in LISTS if "in parts" in name]
 
 
+@pytest.mark.parametrize("name", LISTS)
+@pytest.mark.parametrize("fp32", [False, True])
+def test_rows_of_whole_lines_and_others(name, fp32):
+    """Results whose rows begin with lines of 128 bytes are stored past the caches, others through them: the same bits."""
+    from speculators_amd.gemm import _tn_list
+
+    pairs, dtype = _operands(LISTS[name]), torch.float32 if fp32 else torch.bfloat16
+    got = []
+    for beside, offset in ((8, 0), (8, 8), (0, 0)):
+        lds = [-(-n // 64) * 64 + beside for _, _, n in LISTS[name]]
+        wide = [torch.full((m * ld + 64,), 3.0, device="cuda", dtype=dtype) for (_, m, _), ld in zip(LISTS[name], lds)]
+        outs = [w[offset:offset + m * ld].view(m, ld)[:, :n] for w, (_, m, n), ld in zip(wide, LISTS[name], lds)]
+        assert any(out.data_ptr() % 128 or out.stride(0) * out.element_size() % 128 for out in outs) == (beside > 0)
+        _tn_list(pairs, fp32, outs)
+        assert all((w[offset + m * ld:] == 3).all() and (w[:offset] == 3).all() for w, (_, m, _), ld in zip(wide, LISTS[name], lds))
+        got.append(outs)
+    assert all(torch.equal(a, b) for others in got[1:] for a, b in zip(got[0], others))
+
+
 @pytest.mark.parametrize("dtype,stride", [(torch.float32, 65544), (torch.float32, 1 << 21), (torch.bfloat16, 1 << 22)])
 def test_results_in_rows_far_apart(dtype, stride):
     """A tile's 256 rows of the result span 2 GiB: not on the walking kernel, which offsets them in 32 bits, but as before it."""
