@@ -375,20 +375,25 @@ __global__ __launch_bounds__(256) void gemm_tn_walk_reduce_kernel(List) {
 
 constexpr int kCus = 256;
 
-// us that `wgs` workgroups of `slabs` slabs take, one to a compute unit, fitted to the figures above: 1.39 a slab and, for each, its
-// results (256 KB of them in fp32)
-static float rounds_us(int64_t wgs, int64_t slabs, bool f32) {
+// us that a tile's results take: 128 or 256 KB, and the fp32 ones of a part
+static float results_us(bool f32) { return f32 ? 10.2f : 5.5f; }
+constexpr float kPartUs = 8.f;
+
+// us that `wgs` workgroups of `slabs` slabs take, one to a compute unit.  With the above fitted to 687 products of 130 to 9000 rows,
+// results of 48 to 3000 tiles (4 % rms; 1164 others 4 %, 1 - 3 % too low)
+static float rounds_us(int64_t wgs, int64_t slabs, float results) {
   const int64_t full = wgs / kCus, last = wgs % kCus;
-  return slabs * (full * 1.39f + (last ? 0.95f + 0.44f * last / kCus : 0.f)) + (f32 ? 9.f : 4.f) * (full + (last ? 1 : 0));
+  return full * (slabs * 1.37f + results) + (last ? slabs * (0.86f + 0.37f * last / kCus) + results : 0.f);
 }
 
 // Into how many parts the tiles of the last round are cut (at most kMaxParts, each at least 16 slabs, at most `room` partial
-// tiles): as many as make it shortest, with the pass that adds them (67.5 ns a partial tile).
+// tiles): as many as make it shortest, with the pass that adds them (50 ns a partial tile).  293 last rounds in parts: 1.001 of the
+// better of parts and whole tiles.
 static int tail_of(int rem, int slabs_least, int slabs_most, bool f32, int64_t room, float& us) {
   int best = 1;
-  us = rem ? rounds_us(rem, slabs_most, f32) : 0.f;
+  us = rem ? rounds_us(rem, slabs_most, results_us(f32)) : 0.f;
   for (int p = 2; rem && p <= kMaxParts && slabs_least / p >= 16 && (int64_t)rem * p <= room; ++p) {
-    const float t = rounds_us((int64_t)rem * p, (slabs_most + p - 1) / p, true) + 4.1f + 0.0675f * rem * p;
+    const float t = rounds_us((int64_t)rem * p, (slabs_most + p - 1) / p, kPartUs) + 4.1f + 0.05f * rem * p;
     if (t < 0.97f * us) { us = t; best = p; }
   }
   return best;
@@ -426,8 +431,8 @@ static bool plan(const spx_tn_product* p, int n, bool f32, int64_t room, Plan& o
     const auto& e = p[out.order[k]];
     const int slabs = (int)((e.T + kTK - 1) / kTK);
     at += tiles_of(e.M, e.N);
-    for (; first < std::min(at, tiles - rem); first += kCus) us_first += rounds_us(kCus, slabs, f32);
-    for (; last < std::min(at, tiles - rem); last += kCus) us_last += rounds_us(kCus, slabs, f32);
+    for (; first < std::min(at, tiles - rem); first += kCus) us_first += rounds_us(kCus, slabs, results_us(f32));
+    for (; last < std::min(at, tiles - rem); last += kCus) us_last += rounds_us(kCus, slabs, results_us(f32));
     if (at > tiles - rem) {
       if (!most) most = slabs;
       least = slabs;

@@ -84,6 +84,16 @@ def test_results_in_rows_far_apart(dtype, stride):
     assert (torch.as_strided(out, (8, stride - 65528), (stride, 1), 65528) == 3).all()
 
 
+@pytest.mark.parametrize("t,m,n,fp32,walks", [
+    (1280, 3840, 5376, False, False), (1193, 768, 25088, False, False), (466, 5376, 3648, False, False),  # 1.18 - 1.23 of the smaller tiles
+    (192, 5784, 29112, True, False), (384, 16688, 1816, False, False),  # 1.05
+    (192, 11776, 9192, False, True), (2339, 14448, 3368, False, True), (697, 3520, 7608, True, True)])  # 0.82, 0.92, 0.71
+def test_which_weight_gradients_walk(t, m, n, fp32, walks):
+    from speculators_amd.gemm import _walks
+
+    assert _walks((t, m, n, m, n, n), fp32) == walks
+
+
 def test_rules():
     from speculators_amd import _lib, gemm
 
