@@ -276,9 +276,15 @@ constexpr Config kNN[] = {{256, 256, 1, 0.f, 0.f, 0.f},        // (kFifth)
 // waves takes 6 % longer than the price above.  5 % rms over 40 products of 512 .. 8192 rows -> 896 .. 5000 columns; chosen
 // with it / with the price above, us: 1400 x 8192 -> 4160 92.0 / 96.2, 700 x 11520 -> 2880 54.3 / 57.0, 8192 x 4096 -> 2880 167.0 /
 // 172.7, the other 37 alike: 1.009 of the best candidate in place of 1.013 in the geometric mean.  (Contractions that end
-// inside a slab do not walk either, but there all candidates take as much longer: 30 products a b and 36 a b^T
-// are within 1.02 of the best as they are priced.)
+// inside a slab do not walk either, but there all candidates of this form take as much longer: 30 products are within 1.01 of the
+// best as they are priced.)
 constexpr Config kNNAside = {256, 256, 1, 0.96f, 0.30f, 7.6f};
+// kBig of the first form where no workgroup walks: contractions that end inside a slab or have fewer than three, columns that are no
+// multiple of 8.  A workgroup a tile then pays for the start and the end of each.  316 such products of 200 to 12000 rows, contractions
+// of 64 to 16000: the choice takes 0.974 of that by the walking kernel's price, 0.929 of that before there was one (by more than 3 %
+// slower than that 4, the worst 1.09), and is within 1.023 of the best candidate in place of 1.050.  8288 x 808 -> 2944 62.7 -> 51.3
+// us, 2048 x 1336 -> 17784 113 -> 99.
+constexpr Config kNTAside = {256, 256, 1, 0.90f, 0.30f, 15.f};
 // Weight gradients (contraction slow in both operands): the candidates beside the 256 x 256 kernel of gemm_bf16_tn.hip,
 // which keeps whole rounds of its tiles and is given up only for a predicted tenth.  Fitted the same way to 128 products
 // (results of 1 .. 768 large tiles, 256 .. 20000 rows, up to 12 parts; 6 - 13 % rms).  Over them the choice takes 0.52 of that
@@ -317,7 +323,7 @@ static Choice choose(int form, int64_t M, int64_t N, int64_t K, int max_parts, b
   const Config* const table = nn ? kNN : kNT;
   Choice best{kBig, 1, 1e30f};
   if (!nn) {
-    const Config& c = form == 2 ? kLive : table[kBig];
+    const Config& c = form == 2 ? kLive : K % kTK || K < 3 * kTK || N % 8 ? kNTAside : table[kBig];
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), rem = tiles % kCus;
     int64_t cut = 0;
     int tp = 1;

@@ -453,7 +453,7 @@ def _walking_forward(m: int, n: int, k: int, parts: int | None = None) -> bool:
 
 @functools.lru_cache(maxsize=4096)
 def _walks_as_fast(m: int, n: int, k: int, parts: int) -> bool:
-    if not m or k % 64 or n % 8 or _lib.load().spx_gemm_auto_tile(0, m, n, k, parts):
+    if not m or k % 64 or k < 192 or n % 8 or _lib.load().spx_gemm_auto_tile(0, m, n, k, parts):
         return False
     if k < 4096:
         return True

@@ -70,3 +70,13 @@ def test_routes_go_by_the_parts_that_are_asked_for(monkeypatch):
                                         (1400, 2048, 16384, 5), (8192, 4096, 14336, 5), (3500, 2048, 16384, 5)])
 def test_input_gradients_on_large_tiles(m, n, k, tile):
     assert _lib.load().spx_gemm_auto_tile(1, m, n, k, 4) == tile
+
+
+# a contraction that ends inside a slab, columns that are no multiple of 8, two slabs: no workgroup walks, and the large tile is left; then
+# sizes next to them that are walked
+@pytest.mark.parametrize("m,n,k,large", [(8288, 2944, 808, False), (2048, 17784, 1336, False), (4352, 4288, 72, False),
+                                         (6000, 16384, 128, False), (2048, 17784, 1344, True), (6000, 16384, 192, True)])
+def test_large_tiles_that_do_not_walk(m, n, k, large):
+    assert (_lib.load().spx_gemm_auto_tile(0, m, n, k, 4) == 0) == large
+    if k % 64 == 0:
+        assert gemm._walking_forward(m, n, k) == large
