@@ -10,7 +10,7 @@
 // A workgroup a tile / this, us: 32760 x 2048 -> 12288 1246 / 1130, 1999 x 2048 -> 32000 200 / 187, 4096 x 4096 -> 32000 741 / 715,
 // 4096 x 4096 -> 28672 660 / 623, 4096 x 14336 -> 4096 (one round) 303 / 300, 512 x 2048 -> 32000 (one round) 53.7 / 51.0; in a
 // 1B validation pass 3294 / 3208, an MTP step 171.6 / 169.8 ms.
-// The results leave in whole 128-byte lines, past the caches (STREAM) where they are larger than the 256 MB cache behind them.
+// The results leave in whole 128-byte lines, past the caches (STREAM) where they are larger than the 256 MB cache behind them (walk).
 
 #include <algorithm>
 
@@ -345,6 +345,13 @@ bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, i
          kTM * ldc * 2 < 0x7ffffff0ll && (!slow || (K + 4 * kTK) * ldb * 2 < 0x7ffffff0ll) && n_grid < (1 << 22);
 }
 
+// Results larger than the cache leave past it -- those whose rows do not begin with lines of 64 bytes (tiles share a line at every
+// row, and its pieces go to memory one by one) from contractions on that give the stores the time.  Through the caches / past
+// them, rows at multiples of 16 or 32 bytes: K 192 to 448 0.5 - 1.05 (9204 x 192 -> 21576 122 / 240 us; 0.76 over 37 products), 512 to 896
+// 0.73 - 1.02 (0.91 over 26), 960 to 1216 0.88 - 0.98 over 7, from 1280 on 0.96 - 1.04; rows at multiples of 64 bytes 0.95 - 1.24
+// over 13, of 128 1.01 over 31.
+constexpr int64_t kStreamK = 1280;
+
 template <bool SLOW, bool GRADE, bool STREAM>
 static int launch_walk(const char* fname, const WalkArgs& w, hipStream_t st) {
   static std::atomic<uint64_t> lds_set;
@@ -359,7 +366,8 @@ static int launch_walk(const char* fname, const WalkArgs& w, hipStream_t st) {
 }
 
 int walk(const char* fname, bool slow, const WalkArgs& w, hipStream_t st) {
-  const bool stream = w.M * w.N * 2 > (256ll << 20) && w.parts == 1;
+  const bool lines = w.ldc % 32 == 0 && (uintptr_t)w.c % 64 == 0;
+  const bool stream = w.M * w.N * 2 > (256ll << 20) && w.parts == 1 && (lines || w.K >= kStreamK);
   if (slow) return stream ? launch_walk<true, false, true>(fname, w, st) : launch_walk<true, false, false>(fname, w, st);
   if (w.grade.row) return stream ? launch_walk<false, true, true>(fname, w, st) : launch_walk<false, true, false>(fname, w, st);
   return stream ? launch_walk<false, false, true>(fname, w, st) : launch_walk<false, false, false>(fname, w, st);

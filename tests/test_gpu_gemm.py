@@ -63,6 +63,23 @@ def test_products_of_workgroups_that_walk(m, n, k, live):
         assert ((matmul_nn(a, b.t().contiguous()).float() - ref).abs() <= bound).all()
 
 
+# results of more than 256 MB in rows at multiples of 128, 64 and 16 bytes, on both sides of the contraction from which the last leave
+# past the caches, too
+@pytest.mark.parametrize("n", [15872, 15904, 15880])
+@pytest.mark.parametrize("k", [192, 1216, 1280])
+def test_large_results_of_workgroups_that_walk(n, k):
+    from speculators_amd.gemm import gemm_nt
+
+    m = 8500
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    a, b = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    wide = torch.full((m * n + 64,), 7.0, device="cuda", dtype=torch.bfloat16)
+    gemm_nt(a, b, wide[:m * n].view(m, n))
+    ref = a.float() @ b.float().t()
+    assert ((wide[:m * n].view(m, n).float() - ref).abs() <= 2 ** -8 * (ref.abs() + k ** 0.5)).all()
+    assert (wide[m * n:] == 7).all()
+
+
 @pytest.mark.parametrize("m,n,k,parts", [(1421, 2048, 16384, 5), (2003, 2048, 16384, 4), (1033, 4096, 28672, 3)])
 def test_walking_products_cut_whole(m, n, k, parts):
     """The NN product whose every tile is cut along the contraction, the last part the shortest: fp32 partial results of ragged
