@@ -112,49 +112,78 @@ def test_rules():
         assert rc(**changes) != 0, changes
 
 
-@pytest.mark.parametrize("regime", ["bf16", "autocast", "mixed"])
-def test_a_layer_staged_together(regime):
+class _Into(torch.autograd.Function):
+    """``x`` in a weight's input buffer."""
+
+    @staticmethod
+    def forward(ctx, x, slot):
+        slot.data.copy_(x)  # (as a kernel writes it: the buffer of another use is not "modified")
+        return slot
+
+    @staticmethod
+    def backward(ctx, g):
+        return g, None
+
+
+# one use; two of them in the weights' input buffers: one product a weight either way, and these are one launch for each type of result
+# that several weights have; two uses outside the buffers: a product each, added up
+@pytest.mark.parametrize("regime,lists", [("bf16", {False: 3}), ("autocast", {True: 3}), ("mixed", {False: 2})])
+@pytest.mark.parametrize("uses,slots", [(1, False), (2, True), (2, False)])
+def test_a_layer_staged_together(regime, lists, uses, slots, monkeypatch):
     """The gradients of weights that are staged by one node are those of a node each (the products' sums are the same up to the
     order of fp32 additions), whichever of them are asked for; nothing is kept alive once the graph is gone."""
     import gc
 
+    from speculators_amd import gemm
     from speculators_amd.gemm import linear_staged
     from speculators_amd.weights import WeightStager
 
     torch.manual_seed(1)
     dt = torch.float32 if regime == "autocast" else torch.bfloat16
     new = lambda n, k, d=dt: torch.nn.Parameter((torch.randn(n, k, device="cuda") * k ** -0.5).to(d))  # noqa: E731
-    q, k, o, up = new(512, 512), new(256, 512), new(512, 768), new(1024, 512, torch.float32 if regime == "mixed" else dt)
-    x = torch.randn(600, 512, device="cuda").bfloat16()
+    q, k, o, up = new(1536, 1536, torch.float32 if regime == "mixed" else dt), new(768, 1536), new(1536, 2304), new(3072, 1536)
+    x = torch.randn(600, 1536, device="cuda").bfloat16()
+    launches = []
+    plain = gemm._tn_list
+    monkeypatch.setattr(gemm, "_tn_list", lambda pairs, fp32, outs: launches.append((fp32, len(pairs))) or plain(pairs, fp32, outs))
+
+    def product(h, w):
+        return linear_staged(_Into.apply(h, w.x_slot(600)) if slots else h, w)
 
     def loss(together):
         stager = WeightStager()
-        stager.begin(uses=2)
+        stager.begin(uses=uses)
         with torch.autocast("cuda", torch.bfloat16, enabled=regime != "bf16"):
             if together:
                 wqk, wo, wup = stager.get_all((q, k), (o,), (up,))
             else:
                 wqk, wo, wup = stager.get(q, k), stager.get(o), stager.get(up)
             h = x
-            for _ in range(2):
-                h = linear_staged(linear_staged(linear_staged(h, wqk), wo), wup)[:, :512].contiguous()
+            for _ in range(uses):
+                h = product(product(product(h, wqk), wo), wup)[:, :1536].contiguous()
         return h.float().square().mean()
 
-    torch.backends.cuda.matmul.allow_bf16_reduced_precision_reduction = False
+    monkeypatch.setattr(torch.backends.cuda.matmul, "allow_bf16_reduced_precision_reduction", False)
     params = (q, k, o, up)
     want = torch.autograd.grad(loss(False), params)
+    assert not any(n > 1 for _, n in launches)
     gc.collect()
     gc.disable()
     try:
         before = torch.cuda.memory_allocated()
         for _ in range(3):
+            launches.clear()
             got = torch.autograd.grad(loss(True), params)
+            assert {fp32: n for fp32, n in launches if n > 1} == ({} if uses == 2 and not slots else lists)
+            assert sum(n > 1 for _, n in launches) == (uses == 1 or slots)
             for a, b, p in zip(got, want, params, strict=True):
                 assert a.dtype == p.dtype and (a - b).norm() <= 2 ** -8 * b.norm()
             del got, a
         assert torch.cuda.memory_allocated() == before
         for i, p in enumerate(params):
+            launches.clear()
             part, = torch.autograd.grad(loss(True), (p,))
             assert (part - want[i]).norm() <= 2 ** -8 * want[i].norm()
+            assert not any(n > 1 for _, n in launches)  # (its own product alone)
     finally:
         gc.enable()
