@@ -33,11 +33,11 @@ PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "kernels_config1_hbm_traffic_pmc.txt")
 # bench key -> (substring of the kernel name, launch grid in threads or None = any)
 TRAFFIC_ROWS = {
-    "gemm_fwd": ("gemm_bf16_nt_kernel<true, 0>", 512000),
-    "gemm_dx": ("gemm_bf16_nt_kernel<true, 0>", 65536),
+    "gemm_fwd": ("[gemm_fwd] ", None),
+    "gemm_dx": ("[gemm_dx] ", None),
     "loss_fwd": ("loss_fwd_kernel<unsigned short, 0, true, false, false", None),
     "loss_fwd_reuse": ("loss_fwd_kernel<unsigned short, 0, true, true, false", None),
-    "gemm_tn": ("gemm_bf16_tn_kernel<2, false>", None),
+    "gemm_tn": ("gemm_bf16_tn_walk_kernel<true>", None),
     "loss_fwd_grad_step0": ("loss_fwd_grad_kernel<0, false>", None),
     "loss_fwd_grad": ("loss_fwd_grad_kernel<0, true>", None),
     # (the summary averages the loss backward over its full and packed launches: no per-launch figure)
@@ -493,7 +493,7 @@ def kernel_rooflines(torch, cfg, t, k_steps, device, windows=(None,)):
     xs = torch.randn(k_steps * t, h, device=device, generator=g).bfloat16()
     acc = torch.empty(f2, h, device=device, dtype=torch.float32)
     ms = time_events(torch, lambda: gemm_tn(dys, xs, acc), 5)
-    mfma(f"gemm_bf16_tn_kernel[gate+up weight gradient, all {k_steps} steps: (K T x 2F)^T (K T x H) -> fp32]",
+    mfma(f"gemm_bf16_tn_walk_kernel[gate+up weight gradient, all {k_steps} steps: (K T x 2F)^T (K T x H) -> fp32]",
          2.0 * k_steps * t * f2 * h, ms, 1, "gemm_tn")
     return out
 
@@ -785,11 +785,11 @@ def run_mtp(args):
         xs = torch.randn(pairs_n, h, device=device).bfloat16()
         w_gu = (torch.randn(e, 2 * inter, h, device=device) * 0.02).bfloat16()
         hid = moe.gemm_nt_grouped(xs, w_gu, off)
-        rec("gemm_bf16_nt_kernel[grouped: experts' gate+up, T*k rows x H x 2I, 512 groups]", "mfma",
+        rec("gemm_tile_kernel[grouped: experts' gate+up, T*k rows x H x 2I, 512 groups]", "mfma",
             2.0 * pairs_n * h * 2 * inter, time_events(torch, lambda: moe.gemm_nt_grouped(xs, w_gu, off, out=hid), 3),
             k_steps)
         dw = torch.empty(e, 2 * inter, h, device=device, dtype=torch.float32)
-        rec("gemm_bf16_tn_kernel[grouped: experts' gate+up weight gradient, fp32]", "mfma",
+        rec("gemm_tile_kernel[grouped: experts' gate+up weight gradient, fp32]", "mfma",
             2.0 * pairs_n * h * 2 * inter, time_events(torch, lambda: moe.gemm_tn_grouped(hid, xs, off, dw), 3),
             k_steps)
         xt = torch.randn(tok, h, device=device).bfloat16()
