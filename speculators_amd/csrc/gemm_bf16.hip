@@ -93,10 +93,7 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   // two groups, and the host never learns the group sizes
   if (tile_tab) tiles_m = min(tile_tab[0], tiles_m);
 
-  // workgroup id -> tile index (tile_coords turns that into a tile).  Workgroups go to the eight XCDs round
-  // robin, XCD x gets the ids x, x + 8, ...: they are renumbered so that in every round of 256 workgroups each
-  // XCD has 32 consecutive tile indices, and in what is left after the last whole round one contiguous piece
-  // (the first n % 8 XCDs one more).
+  // workgroup id -> tile index (xcd_order; tile_coords turns that into a tile).
   // contraction in parts (part_ws): the workgroups of part p multiply columns [p, p + 1) * part length of
   // K and leave an fp32 partial in part_ws[p]; gemm_splitk_reduce_kernel adds the parts in order
   const int n_tiles = tiles_m * tiles_n;
@@ -110,20 +107,9 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
   const int n_tail = n_tiles - tail_first;
   const int n_wg = tail_mode ? n_tiles + n_tail * (tail_parts - 1) : n_tiles * parts;
   if ((int)blockIdx.x >= n_wg) return;
-  int pid;
-  {
-    constexpr int kRound = 256, kPer = kRound / 8;
-    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-    // (with a cut last round the whole tiles are whole rounds, and the parts of the cut ones are rounds of their own behind
-    // them: workgroups start in the order of their ids)
-    const int full = n_wg / kRound * kRound;
-    if ((int)blockIdx.x < full) {
-      pid = (local / kPer) * kRound + xcd * kPer + local % kPer;
-    } else {
-      const int nr = n_wg - full;
-      pid = full + xcd * (nr >> 3) + min(xcd, nr & 7) + (local - full / 8);
-    }
-  }
+  // (with a cut last round the whole tiles are whole rounds, and the parts of the cut ones are rounds of their own behind
+  // them: workgroups start in the order of their ids)
+  int pid = xcd_order(blockIdx.x, n_wg);
   int part;
   if (tail_mode) {
     part = 0;

@@ -30,7 +30,7 @@
 // matrix pipe.  Before / now, us: 28672 rows -> 4096 x 28672 4768 / 4517 (1491 TFLOP/s), -> 4096 x 14336 2633 / 2457,
 // -> 6144 x 8192 2026 / 1936; 98280 -> 6144 x 2048 2029 / 1896; 32000 -> 12288 x 2048 1356 / 1247; 1536 -> 16384 x 2048 92.5 / 90.7.
 
-#include "gemm_tile_api.h"
+#include "gemm_nt.h"
 #include "spx_common.h"
 #include "../../include/spx.h"
 
@@ -121,36 +121,8 @@ __global__ __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(1, 
   // the operand on that side is read in one round only, the other operand again every round.  Inside a round
   // each XCD (workgroups go to them round robin) has 32 neighbouring tiles, 8 along the longer side x 4: 12
   // bands through its L2, and a band of the longer side's operand is shared by four XCDs at the same time.
-  const int n_wg = tiles_m * tiles_n;
-  int pid;
-  {
-    constexpr int kRound = 256, kPer = kRound / 8;
-    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-    const int full = n_wg / kRound * kRound;
-    if ((int)blockIdx.x < full) {
-      pid = (local / kPer) * kRound + xcd * kPer + local % kPer;
-    } else {  // the last, partial round: one contiguous piece per XCD (the first n % 8 get one tile more)
-      const int nr = n_wg - full, base = nr >> 3, rem = nr & 7;
-      pid = full + xcd * base + min(xcd, rem) + (local - full / 8);
-    }
-  }
   int tile_m, tile_n;
-  {
-    // tiles in the order of pid: panels of kPanel along the shorter side; inside a panel groups of kGroup along
-    // the longer side; inside a group the longer side first (the NT kernel's tile_coords: same order)
-    constexpr int kPanel = 16, kGroup = 8;
-    const bool m_long = tiles_m >= tiles_n;
-    const int tl = m_long ? tiles_m : tiles_n, ts = m_long ? tiles_n : tiles_m;
-    const int panel = pid / (tl * kPanel);
-    const int ps = min(ts - panel * kPanel, kPanel);
-    const int p = pid - panel * tl * kPanel;
-    const int g = p / (kGroup * ps);
-    const int gsz = min(tl - g * kGroup, kGroup);
-    const int r = p - g * kGroup * ps;
-    const int l = g * kGroup + r % gsz, sh = panel * kPanel + r / gsz;
-    tile_m = m_long ? l : sh;
-    tile_n = m_long ? sh : l;
-  }
+  tile_coords(xcd_order(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tile_m, tile_n);
   const int m0 = tile_m * kTM, n0 = tile_n * kTN;
 
   const int tid = threadIdx.x, lane = tid & 63;

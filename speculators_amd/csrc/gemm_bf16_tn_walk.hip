@@ -80,16 +80,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) __attribute__((amdgpu_waves_per_eu
     Tile t{};
     t.part = -1;
     if (id >= n_wg) return t;  // nothing: its loads bring zeros
-    // the ids go to the eight XCDs round robin: 32 consecutive tiles per XCD and round, a contiguous piece of what is left
-    constexpr int kRound = 256, kPer = kRound / 8;
-    const int xcd = id & 7, local = id >> 3, full = n_wg / kRound * kRound;
-    int pid;
-    if (id < full) {
-      pid = (local / kPer) * kRound + xcd * kPer + local % kPer;
-    } else {
-      const int nr = n_wg - full;
-      pid = full + xcd * (nr >> 3) + min(xcd, nr & 7) + (local - full / 8);
-    }
+    int pid = xcd_order(id, n_wg);
     int part = 0, parts = 1;
     if (tail_parts > 1 && pid >= tail_first) {
       const int qq = pid - tail_first;

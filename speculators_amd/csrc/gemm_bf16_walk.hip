@@ -72,16 +72,7 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
       t.bres = make_rsrc(B, 0);
       return t;
     }
-    // the ids go to the eight XCDs round robin: 32 consecutive tiles per XCD and round, a contiguous piece of what is left
-    constexpr int kRound = 256, kPer = kRound / 8;
-    const int xcd = id & 7, local = id >> 3, full = n_wg / kRound * kRound;
-    int pid;
-    if (id < full) {
-      pid = (local / kPer) * kRound + xcd * kPer + local % kPer;
-    } else {
-      const int nr = n_wg - full;
-      pid = full + xcd * (nr >> 3) + min(xcd, nr & 7) + (local - full / 8);
-    }
+    int pid = xcd_order(id, n_wg);
     int k0 = 0;
     t.slabs = all_slabs;
     t.part = -1;
@@ -341,8 +332,12 @@ __attribute__((amdgpu_waves_per_eu(SPX_GEMM_MINW, SPX_GEMM_MINW))) void gemm_bf1
 
 bool walk_takes(bool slow, const void* c, int64_t ldb, int64_t ldc, int64_t N, int64_t K, int64_t n_grid, int parts) {
   const int64_t slabs = K / kTK, per = (slabs + parts - 1) / parts;
-  return K % kTK == 0 && per >= 3 && slabs - per * (parts - 1) >= 3 && (parts == 1 || kTM * N * 4 < 0x7ffffff0ll) && N % (slow ? kTN : 8) == 0 && ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0 &&
-         kTM * ldc * 2 < 0x7ffffff0ll && (!slow || (K + 4 * kTK) * ldb * 2 < 0x7ffffff0ll) && n_grid < (1 << 22);
+  const bool slabs_enough = K % kTK == 0 && per >= 3 && slabs - per * (parts - 1) >= 3;  // (of the last part, too)
+  const bool whole_pieces = N % (slow ? kTN : 8) == 0 && ldc % 8 == 0 && ((uintptr_t)c) % 16 == 0;
+  // (32-bit offsets inside a tile of c or of partial results, and of B where it is read down its rows)
+  const bool spans = kTM * ldc * 2 < 0x7ffffff0ll && (parts == 1 || kTM * N * 4 < 0x7ffffff0ll) &&
+                     (!slow || (K + 4 * kTK) * ldb * 2 < 0x7ffffff0ll);
+  return slabs_enough && whole_pieces && spans && n_grid < (1 << 22);
 }
 
 // Results larger than the cache leave past it -- those whose rows do not begin with lines of 64 bytes (tiles share a line at every

@@ -91,6 +91,17 @@ __device__ __forceinline__ int small_div(int a, int b) {
   return __builtin_amdgcn_readfirstlane(q);
 }
 
+// workgroup id -> place in the order of the work.  Workgroups go to the eight XCDs round robin, XCD x gets the ids x, x + 8, ...: they
+// are renumbered so that in every round of 256 workgroups each XCD has 32 consecutive places, and in what is left after the last whole
+// round one contiguous piece (the first n % 8 XCDs one more).
+__device__ __forceinline__ int xcd_order(int id, int n_wg) {
+  constexpr int kRound = 256, kPer = kRound / 8;
+  const int xcd = id & 7, local = id >> 3, full = n_wg / kRound * kRound;
+  if (id < full) return (local / kPer) * kRound + xcd * kPer + local % kPer;
+  const int nr = n_wg - full;
+  return full + xcd * (nr >> 3) + min(xcd, nr & 7) + (local - full / 8);
+}
+
 // tile index -> (tile row, tile column).  256 consecutive indices (what the chip runs at a time) are a block of
 // 16 x 16 tiles, so that a 256-row band of either operand is used by 16 of the tiles in flight, and the blocks walk
 // along the longer side of the tile grid; 32 consecutive indices (what one XCD runs: see the kernel) are 8 tiles
