@@ -89,7 +89,7 @@ CONFIG1 = dict(hidden_size=4096, num_attention_heads=32, num_key_value_heads=8, 
                rope_scaling={"rope_type": "llama3", "factor": 8.0, "low_freq_factor": 1.0,
                              "high_freq_factor": 4.0, "original_max_position_embeddings": 8192})
 SEQ_LEN, TTT_STEPS = 4096, 7
-# the Llama-3.1-70B shape (seq 8192, TTT 5), same code path as configs[1]
+# the Llama-3.1-70B shape (seq 8192, TTT 5), same code path as the 8B one
 CONFIG3 = dict(CONFIG1, hidden_size=8192, num_attention_heads=64, intermediate_size=28672)
 SEQ_LEN3, TTT_STEPS3 = 8192, 5
 
@@ -99,9 +99,9 @@ def parse_args():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--workload", choices=["eagle3", "eagle3-70b", "mtp", "mtp-next", "dflash"],
                     default="eagle3",
-                    help="eagle3 = configs[1], the headline; eagle3-70b = configs[3]; mtp = configs[4] (MTP "
-                         "head, full-vocab CE); mtp-next = the same shape with the qwen3_next layer (gated "
-                         "attention, partial rotary, 512-expert MoE); dflash = configs[2] (anchored blocks, "
+                    help="eagle3 = the Llama-3.1-8B shape, the headline; eagle3-70b = the 70B shape; mtp = the MTP head "
+                         "(full-vocab CE); mtp-next = the same shape with the qwen3_next layer (gated "
+                         "attention, partial rotary, 512-expert MoE); dflash = the Qwen3-8B shape (anchored blocks, "
                          "5 layers)")
     ap.add_argument("--steps", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=5)
@@ -119,8 +119,8 @@ def parse_args():
                          "gradients (the regime of the reference's Trainer, train/trainer.py:459-465); "
                          "bf16: the whole model cast to bf16 (the reference's integration tests)")
     ap.add_argument("--window", type=int, default=0,
-                    help="sliding window of every draft layer for the HEADLINE figure (0 = full attention, what "
-                         "BASELINE's configs[1] names).  The reference's scripts/train.py makes every EAGLE3 draft "
+                    help="sliding window of every draft layer for the HEADLINE figure (0 = full attention). "
+                         "The reference's scripts/train.py makes every EAGLE3 draft "
                          "layer sliding-window with W = 2048 unless --full-attention-indices is given "
                          "(scripts/train.py:176-179,498-506; train/config/schema.py:172-183): the default run "
                          "times that configuration as a second figure, `reference_default_config`")
@@ -563,7 +563,7 @@ def _hip_same_case(torch, device, cfg, w, case, k_steps):
 
 def cpu_baseline(torch, device, cfg, t, k_steps):
     """The oracle (CPU restatement of the reference eager path, fp32) timed on the host cores:
-    configs[0] in full (1 warm-up + 3 timed forward + backward), and one forward + backward of
+    the Llama-3.2-1B shape in full (1 warm-up + 3 timed forward + backward), and one forward + backward of
     the headline shape on a shortened sequence.  Both cases also go through the HIP model with the
     same weights and inputs: an in-run parity check (loss, exact mask counts)."""
     cores = os.cpu_count() or 1
@@ -577,7 +577,7 @@ def cpu_baseline(torch, device, cfg, t, k_steps):
                 "rel": round(abs(gl - cpu_loss) / abs(cpu_loss), 7),
                 "counts_equal": all(gm[k] == float(cpu_metrics[k]) for k in totals)}
 
-    # the reference's own CPU-runnable case, in full
+    # the Llama-3.2-1B shape: the reference's own CPU-runnable case, in full
     shape0, w0, case0 = _oracle_case(torch, CONFIG0, SEQ_LEN0, 1.0)
     _oracle_step(torch, shape0, w0, case0, TTT_STEPS0)
     times = []
@@ -586,7 +586,7 @@ def cpu_baseline(torch, device, cfg, t, k_steps):
         times.append(dt)
     mean0 = sum(times) / len(times)
     std0 = (sum((x - mean0) ** 2 for x in times) / len(times)) ** 0.5
-    cfg0 = {"workload": f"configs[0]: Llama-3.2-1B shape, seq {SEQ_LEN0}, TTT {TTT_STEPS0}, fp32, in full",
+    cfg0 = {"workload": f"Llama-3.2-1B shape, seq {SEQ_LEN0}, TTT {TTT_STEPS0}, fp32, in full",
             "value": round(SEQ_LEN0 / mean0, 2), "unit": "tokens/s",
             "s_per_iteration": round(mean0, 3), "s_std": round(std0, 3), "iterations": "1 warm-up + 3 timed",
             "parity": parity(_hip_same_case(torch, device, CONFIG0, w0, case0, TTT_STEPS0), loss0, m0)}
@@ -598,12 +598,12 @@ def cpu_baseline(torch, device, cfg, t, k_steps):
     par = parity(_hip_same_case(torch, device, cfg, w, case, k_steps), loss, m)
     return {"value": round(t / dt, 2), "unit": "tokens/s", "cores": threads, "kind": "port",
             "cpu_model": _cpu_model_name(), "host_cpus": cores,
-            "sample": f"config[1] shape (Llama-3.1-8B draft, TTT {k_steps}, fp32 oracle), sequence "
+            "sample": f"Llama-3.1-8B draft shape (TTT {k_steps}, fp32 oracle), sequence "
                       f"shortened to {t} tokens, 1 forward+backward, no warm-up, {dt:.1f} s",
-            "parity": par, "configs0": cfg0}
+            "parity": par, "llama_1b_in_full": cfg0}
 
 
-# configs[4]: MTP head finetune, Qwen3-Next-like shape.  The FFN width is not stated there;
+# MTP head finetune, Qwen3-Next-like shape.  The FFN width is not stated there;
 # 3 x hidden is assumed.  The layer built is the Qwen3 flavour of the MTP layer.
 CONFIG4 = dict(hidden_size=2048, num_attention_heads=16, num_key_value_heads=2, head_dim=256,
                intermediate_size=6144, vocab_size=151936, rms_norm_eps=1e-6, rope_theta=1000000.0)
@@ -614,7 +614,7 @@ NEXT_EXTRA = dict(model_type="qwen3_next", partial_rotary_factor=0.25, num_exper
 
 
 def run_mtp(args):
-    """configs[4]: MTP forward + backward, tokens/s over all B x T positions, and the roofline of
+    """MTP forward + backward, tokens/s over all B x T positions, and the roofline of
     the label cross-entropy kernels, the full-vocabulary lm_head GEMMs and the attention."""
     import torch
 
@@ -838,7 +838,7 @@ def run_mtp(args):
         cpu_step()
         cdt = time.perf_counter() - c0
         cpu = {"value": round(b * tn / cdt, 2), "unit": "tokens/s", "cores": torch.get_num_threads(),
-               "kind": "port", "sample": f"oracle MTP forward+backward, configs[4] shape at batch {b} x seq {tn}, "
+               "kind": "port", "sample": f"oracle MTP forward+backward, the timed shape at batch {b} x seq {tn}, "
                                          + ("fp32, qwen3_next layer with 512 experts (8 random ones tiled), one timed "
                                             "iteration, no warm-up" if hybrid else
                                             "fp32, 1 warm-up + 1 timed iteration")}
@@ -848,11 +848,11 @@ def run_mtp(args):
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms_per_step, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "bf16",
         "data": "synthetic",
-        "config": {"workload": (f"configs[4] shape with the qwen3_next layer: gated attention, rotary on 64 of 256, "
+        "config": {"workload": (f"MTP head with the qwen3_next layer: gated attention, rotary on 64 of 256, "
                                 f"512 experts top-10 of width 512 + shared expert 512, hidden 2048, 16 q / 2 kv "
                                 f"heads, head_dim 256, vocab 151936, batch {b}, seq {n}, {k_steps} prediction "
                                 f"steps, label cross-entropy, loss_mask Bernoulli(0.7)") if hybrid else
-                               f"configs[4]: MTP head, one Qwen3 decoder layer, hidden 2048, 16 q / 2 kv heads, "
+                               f"MTP head, one Qwen3 decoder layer, hidden 2048, 16 q / 2 kv heads, "
                                f"head_dim 256, FFN 6144 (assumed), vocab 151936, batch {b}, seq {n}, "
                                f"{k_steps} prediction steps, label cross-entropy, loss_mask Bernoulli(0.7)",
                    "seq_len": n, "batch": b, "steps": k_steps, "tokens_per_step": tokens,
@@ -863,7 +863,7 @@ def run_mtp(args):
         "kernels": kernels, "cpu_baseline": cpu}))
 
 
-# configs[2]: DFlash on a Qwen3-8B shaped verifier.  5 draft layers (the reference default for
+# DFlash on a Qwen3-8B shaped verifier.  5 draft layers (the reference default for
 # dflash), every layer windowed; 512 anchors on a uniform non-overlapping grid.
 CONFIG2 = dict(hidden_size=4096, num_attention_heads=32, num_key_value_heads=8, head_dim=128,
                intermediate_size=12288, vocab_size=151936, draft_vocab_size=32000, num_aux=5,
@@ -873,7 +873,7 @@ DFLASH_SEQ_LEN, DFLASH_ANCHORS = 8192, 512
 
 
 def run_dflash(args):
-    """configs[2]: DFlash forward + backward, tokens/s over the T context positions, and the
+    """DFlash forward + backward, tokens/s over the T context positions, and the
     roofline of the anchored-block attention."""
     import torch
 
@@ -964,7 +964,7 @@ def run_dflash(args):
         "unit": "tokens/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": round(ms_per_step, 3), "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
-        "config": {"workload": f"configs[2]: DFlash draft, Qwen3-8B shape, {cfg.num_hidden_layers} layers, seq {t}, "
+        "config": {"workload": f"DFlash draft, Qwen3-8B shape, {cfg.num_hidden_layers} layers, seq {t}, "
                                f"{n_anchor} anchors x block {bs} (queries {n_q}, keys {t + n_q}), window {w} on "
                                "every layer, 5 auxiliary layers, vocab 151936 -> draft 32000, kl_div loss",
                    "seq_len": t, "anchors": n_anchor, "block_size": bs, "tokens_per_step": t,
@@ -1068,7 +1068,7 @@ def main():
                        "ms_per_step": round(w_ms, 3), "value": round(t / (w_ms * 1e-3), 1), "unit": "tokens/s",
                        "final_loss": round(float(loss.detach()), 6),
                        "note": "what scripts/train.py trains by default (scripts/train.py:176-179,498-506); "
-                               "BASELINE's configs[1] names no window, so the headline above is full attention"}
+                               "the headline above is full attention"}
         del model, step, loss
         torch.cuda.empty_cache()
 
@@ -1144,8 +1144,8 @@ def main():
         "value": round(value, 1), "unit": "tokens/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": round(ms_per_step, 3), "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
-        "config": {"workload": ("configs[3]: EAGLE3 draft, Llama-3.1-70B shape, one draft layer, " if big else
-                                "configs[1]: EAGLE3 draft, Llama-3.1-8B shape, one draft layer, ")
+        "config": {"workload": ("EAGLE3 draft, Llama-3.1-70B shape, one draft layer, " if big else
+                                "EAGLE3 draft, Llama-3.1-8B shape, one draft layer, ")
                                +
                                f"batch 1, seq {t}, TTT {k_steps}, vocab 128256 -> draft 32000, "
                                f"{args.loss} loss, "

@@ -180,7 +180,7 @@ def test_model_forward_backward_matches_oracle(weighting, sliding, head_dim):
 
 
 def test_full_size_sampled_rows():
-    """configs[2] shape (seq 8192, 512 anchors x block 16 -> 8192 queries, 16384 keys, window
+    """The Qwen3-8B shape (seq 8192, 512 anchors x block 16 -> 8192 queries, 16384 keys, window
     2048, 32 q / 8 kv heads, head_dim 128): sampled rows (forward and dQ) against the explicit
     fp32 soft-max over the keys the mask rule of models/dflash/attention.py:7-100 lets each row
     see, and the dV column-sum identity."""

@@ -358,7 +358,7 @@ def test_full_size_rows_properties():
 
 
 def test_full_size_row_pass_with_gradient_properties():
-    """The one-read row pass at the config[1] row shape (4096 x 32000 bf16, 70 % of the rows live, target
+    """The one-read row pass at the 8B draft's row shape (4096 x 32000 bf16, 70 % of the rows live, target
     statistics of an earlier step handed in): against the streaming kernels on the same rows -- arg-maxes,
     counts and chain identical, row losses within 1e-5 -- and through what needs no oracle at size: KL rows
     >= 0, every gradient row sums to ~0 (two soft-maxes), the gradient of a row paired with itself is zero,
