@@ -906,7 +906,7 @@ typedef struct spx_tn_product {
 /* 1 .. 8 weight gradients in one launch, bf16 or (out_f32) fp32: the 256 x 256 tiles of all of them are walked by one workgroup
  * per compute unit, products of long contractions first, and those of the last round are cut along the contraction where that
  * is shorter and `workspace` (16-byte aligned, may be NULL) holds their fp32 partial results; these are added in a fixed order.
- * Rules of the two entry points above, but operands of any span; and T at least 129, lda and ldb at least 256, c 16-byte aligned
+ * Rules of the two entry points above, but operands of any span; and T from 129 to 2^28 - 576, lda and ldb at least 256, c 16-byte aligned
  * with a leading dimension that is a multiple of 8 (spx_gemm_tn_list_us: microseconds it is predicted to take, -1 where it is
  * not taken).  spx_gemm_tn_list_workspace_bytes: what the workspace has to hold to be used. */
 int64_t spx_gemm_tn_list_workspace_bytes(const spx_tn_product* products, int n, int out_f32);

@@ -403,7 +403,8 @@ static bool plan(const spx_tn_product* p, int n, bool f32, int64_t room, Plan& o
   if (n < 1 || n > kMaxItems) return false;
   int64_t tiles = 0;
   for (int i = 0; i < n; ++i) {
-    if (p[i].T <= 2 * kTK || p[i].lda < kTM || p[i].ldb < kTN || p[i].ldc % 8 || (uintptr_t)p[i].c % 16 ||
+    // (the kernel divides slabs and parts by small_div)
+    if (p[i].T <= 2 * kTK || (p[i].T + kTK - 1) / kTK + kMaxParts >= 1 << 22 || p[i].lda < kTM || p[i].ldb < kTN || p[i].ldc % 8 || (uintptr_t)p[i].c % 16 ||
         kTM * p[i].ldc * (f32 ? 4 : 2) >= 0x7ffffff0ll || kTK * p[i].lda * 2 >= 0x7ffffff0ll || kTK * p[i].ldb * 2 >= 0x7ffffff0ll)
       return false;
     tiles += tiles_of(p[i].M, p[i].N);

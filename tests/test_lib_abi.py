@@ -164,3 +164,11 @@ def test_a_pair_product_cut_whole_needs_its_workspace(workspace, room):
     assert lib.spx_gemm_pair_takes(1, m, n, k, n, 4) and lib.spx_gemm_auto_workspace_bytes(1, m, n, k, 4) > 1 << 20
     rc = lib.spx_gemm_bf16_pair(1, 4096, k, 4096, 4096, n, 4096, n, m, n, k, 4, workspace, room, None, None)
     assert rc == 1 and b"workspace" in lib.spx_last_error()
+
+
+@pytest.mark.parametrize("rows,taken", [(128, False), (129, True), ((1 << 28) - 576, True), ((1 << 28) - 575, False), (1 << 28, False)])
+def test_contractions_that_workgroups_walk(rows, taken):
+    """Three slabs at least, and with eight parts fewer than 2^22: the kernel divides their number by a reciprocal good to there."""
+    from speculators_amd import gemm
+
+    assert (gemm._tn_list_plan(((rows, 4096, 4096, 4096, 4096, 4096),), True)[0] > 0) == taken
