@@ -15,8 +15,6 @@
 
 namespace spx {
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
 constexpr int kAttnThreads = 256;
 constexpr int kBM = 128;  // query rows per workgroup
 constexpr int kBN = 64;   // keys per tile
@@ -46,15 +44,6 @@ __device__ __forceinline__ bf16x8 pack8(const f32x16& a, int base) {
   c.u.z = pack_bf16x2(a[base + 4], a[base + 5]);
   c.u.w = pack_bf16x2(a[base + 6], a[base + 7]);
   return c.b;
-}
-
-template <typename T>
-__device__ __forceinline__ T lds_get(uint32_t addr) {
-  return *reinterpret_cast<const __attribute__((address_space(3))) T*>((uintptr_t)addr);
-}
-template <typename T>
-__device__ __forceinline__ void lds_put(uint32_t addr, T v) {
-  *reinterpret_cast<__attribute__((address_space(3))) T*>((uintptr_t)addr) = v;
 }
 
 // dot product of two 8-element bf16 fragments, accumulated in fp32 with the packed

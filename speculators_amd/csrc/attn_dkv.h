@@ -69,6 +69,14 @@ typedef __attribute__((ext_vector_type(4))) int i32x4;
 __device__ __forceinline__ f32x4 mfma16b(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+template <typename T>
+__device__ __forceinline__ T lds_get(uint32_t addr) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) T*>((uintptr_t)addr);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(uint32_t addr, T v) {
+  *reinterpret_cast<__attribute__((address_space(3))) T*>((uintptr_t)addr) = v;
+}
 
 // What both roles know about the workgroup's work; every value is wave-uniform.
 struct DkvJob {

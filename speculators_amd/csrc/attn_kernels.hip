@@ -342,25 +342,23 @@ struct PrioPair {
 // that pipe busy all the time.  The transposed operand of the second product comes out of the row-major tile through
 // transposing LDS reads (dQ: K^T; forward, TR: V^T), or, in larger forward calls, out of a copy V^T made once per call: two
 // 8-byte reads for one of 16 cost the forward 5 - 6 %, the copy is a launch of 4 us (fwd_tr).
-// KS: groups of NW waves over the same rows, each with every KS-th tile and two buffers of its own (few_workgroups).
-template <int D, int NW, int KS = 1>
+template <int D, int NW>
 struct FwdSmem {
   static constexpr int kTile = kBN * D * 2;  // unpadded, swizzled
   static constexpr int kBuf = 2 * kTile;     // K, V
-  static constexpr int kTiles = KS * 2 * kBuf;
-  static constexpr int kBytes = kTiles + (KS > 1 ? NW * KS * 512 : 4 * NW * (int)sizeof(int));
+  static constexpr int kTiles = 2 * kBuf;
+  static constexpr int kBytes = kTiles + 4 * NW * (int)sizeof(int);
 };
 
 // operand fragments in flight per product (registers: 4 per fragment): the LDS pipe delivers
 // well over 150 B/clk per CU, what a wave waits for is the latency of its own reads
 #define SPX_FWD_RING 8
-template <int D, int NSB, int NW, bool TR, int KS = 1>
-__global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_kernel(AttnParams p,
+template <int D, int NSB, int NW, bool TR>
+__global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_FWD_MINB) void attn_fwd_kernel(AttnParams p,
                                                                 const uint16_t* __restrict__ Vt,
                                                                 uint16_t* __restrict__ O,
                                                                 float* __restrict__ LSE) {
-  static_assert(KS == 1 || (TR && NSB == 1 && D <= 128), "groups of waves: few_workgroups");
-  using SM = FwdSmem<D, NW, KS>;
+  using SM = FwdSmem<D, NW>;
   constexpr int NKK = D / 16;
   constexpr int NDB = D / 32;
   constexpr int BMW = 32 * NSB;
@@ -379,8 +377,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
   const int m0 = qb * BM;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // in a scalar register: what derives from it is scalar too
-  const int wave = KS > 1 ? wave_all % NW : wave_all, grp = KS > 1 ? wave_all / NW : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in a scalar register: what derives from it is scalar too
   const int g = lane >> 5, col = lane & 31;
   int i[NSB], ic[NSB];
 #pragma unroll
@@ -389,7 +386,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
     ic[sb] = i[sb] < p.NQ ? i[sb] : p.NQ - 1;
   }
   RowBounds<NSB> rb;
-  load_bounds<NSB, NW * KS>(p, ic, wave_all, lane, red, rb);
+  load_bounds<NSB, NW>(p, ic, wave, lane, red, rb);
 
   // The query fragments carry the soft-max scale and log2(e): the scores then come out of the
   // MFMA in the base-2 exponent domain and need no multiply of their own.
@@ -436,8 +433,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
   constexpr int LPK = (kBN * RBK / 1024) / NW;           // wave loads per wave and tile
   auto swz_k = [](int r) { return CKK == 8 ? (r >> 1) & 7 : r & 15; };
   auto swz_v = [](int r) { return CKK == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3); };
-  const uint32_t lds_all = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)fwd_smem;
-  const uint32_t lds0 = lds_all + grp * (2 * SM::kBuf);  // this group's tile buffers
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)fwd_smem;
   const u32x4 kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
   const uint16_t* const Vth = Vt + (int64_t)kvh * D * p.NKVp;
   const u32x4 vres = TR ? make_rsrc(Vh, (uint32_t)((int64_t)p.NKV * RBK))
@@ -539,16 +535,16 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
   auto run_pass = [&](const int (&aa)[NSB], const int (&bb)[NSB], int w_amin, int w_amax,
                       int w_bmin, int w_bmax, int blk_a, int blk_b) {
     if (blk_b <= blk_a) return;
-    const int n_first = (blk_a / kBN) * kBN, n_begin = n_first + grp * kBN;
+    const int n_begin = (blk_a / kBN) * kBN;
     __syncthreads();  // a previous pass may still be reading either buffer
-    if (KS == 1 || n_begin < blk_b) issue(n_begin, 0);
+    issue(n_begin, 0);
     auto tile = [&](int n0, auto buf_c) __attribute__((always_inline)) {
       constexpr int buf = decltype(buf_c)::value;
       // this wave's loads of tile n0 have landed; after the barrier everybody's have, and nobody
       // reads the other buffer any more: the next tile goes there
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (n0 + KS * kBN < blk_b) issue(n0 + KS * kBN, buf ^ 1);
+      if (n0 + kBN < blk_b) issue(n0 + kBN, buf ^ 1);
       if (n0 >= w_bmax || n0 + kBN <= w_amin) return;  // nothing visible for this wave
 
       f32x16 st[NSB][2];
@@ -672,10 +668,9 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
       }
       SPX_FWD_PRIO_VALU();
     };
-    // (every group takes as many turns as the first, and waits at the same barriers: past the last tile there is nothing to see)
-    for (int n0 = n_first; n0 < blk_b; n0 += 2 * KS * kBN) {
-      tile(n0 + grp * kBN, std::integral_constant<int, 0>{});
-      if (n0 + KS * kBN < blk_b) tile(n0 + (KS + grp) * kBN, std::integral_constant<int, 1>{});
+    for (int n0 = n_begin; n0 < blk_b; n0 += 2 * kBN) {
+      tile(n0, std::integral_constant<int, 0>{});
+      if (n0 + kBN < blk_b) tile(n0 + kBN, std::integral_constant<int, 1>{});
     }
   };
 
@@ -1006,9 +1001,9 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
     constexpr int XCK = RBK / 16;                  // 16-byte chunks per row
     constexpr int XRL = 1024 / RBK;                // rows per 1 KB wave load
     constexpr int XNL = 32 / XRL;                  // wave loads per 32 rows
-    static_assert(SM::kTiles / (NW * KS) >= 2 * 32 * RBK, "a wave's share of the tile buffers holds K and V rows");
+    static_assert(SM::kTiles / NW >= 2 * 32 * RBK, "a wave's share of the tile buffers holds K and V rows");
     __syncthreads();  // every wave is done with the tile buffers
-    const uint32_t xk = lds_all + wave_all * (2 * 32 * RBK), xv = xk + 32 * RBK;
+    const uint32_t xk = lds0 + wave * (2 * 32 * RBK), xv = xk + 32 * RBK;
     const int64_t kv_bytes = (int64_t)(p.n_extra + 1) * p.T * RBK;
     const u32x4 xkres = make_rsrc(p.K + (int64_t)kvh * p.k_hs, (uint32_t)kv_bytes);
     const u32x4 xvres = make_rsrc(p.V + (int64_t)kvh * p.v_hs, (uint32_t)kv_bytes);
@@ -1024,14 +1019,12 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
 #pragma unroll
       for (int n = 0; n < XNL; ++n) load_to_lds16<0>(res, dst + n * 1024, goff[n], soff);
     };
-    const uint8_t* const xkp = fwd_smem + wave_all * (2 * 32 * RBK);
+    const uint8_t* const xkp = fwd_smem + wave * (2 * 32 * RBK);
     const uint8_t* const xvp = xkp + 32 * RBK;
     const int xrow = col * RBK, xsw = col & (XCK - 1);
-    if (KS == 1 || grp < p.n_extra) {
-      issue_x(xkres, xk, 1 + grp);
-      issue_x(xvres, xv, 1 + grp);
-    }
-    for (int j = 1 + grp; j <= p.n_extra; j += KS) {
+    issue_x(xkres, xk, 1);
+    issue_x(xvres, xv, 1);
+    for (int j = 1; j <= p.n_extra; ++j) {
       // K rows of step j have landed (the V rows, issued after them, may still be in flight)
       if constexpr (XNL == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
       else if constexpr (XNL == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
@@ -1042,7 +1035,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
         dot = dot8_bf16(qf[0][kk], *reinterpret_cast<const u32x4*>(xkp + xrow + (((2 * kk + g) ^ xsw) * 16)), dot);
       const float sj = half_swap_sum(dot);  // the query fragments carry the scale
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // V rows landed, K rows read
-      if (j + KS <= p.n_extra) issue_x(xkres, xk, j + KS);
+      if (j < p.n_extra) issue_x(xkres, xk, j + 1);
       const float m_new = fmaxf(m_run[0], sj);
       const float alpha = fast_exp2(m_run[0] - m_new);  // a row without context keys: exp2(-inf) = 0
       const float pv = fast_exp2(sj - m_new);
@@ -1058,58 +1051,11 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_FWD_MINB) void attn
           for (int t = 0; t < 4; ++t)
             acc[0][db][r4 * 4 + t] = fmaf(pv, vv[t], acc[0][db][r4 * 4 + t] * alpha);
         }
-      if (j + KS <= p.n_extra) {
+      if (j < p.n_extra) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // V rows read
-        issue_x(xvres, xv, j + KS);
+        issue_x(xvres, xv, j + 1);
       }
     }
-  }
-
-  if constexpr (KS > 1) {
-    // the groups' sums meet in the first: each in its wave's share of the tile buffers, reference and row sum behind them
-    __syncthreads();
-    const uint32_t share = lds_all + wave_all * (NDB * 4096) + lane * 16, stat = lds_all + SM::kTiles + wave_all * 512 + lane * 8;
-    static_assert(NW * KS * NDB * 4096 <= SM::kTiles, "32 rows x D sums a wave");
-    if (grp > 0) {
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          lds_put<f32x4>(share + (db * 4 + q) * 1024, f32x4{acc[0][db][4 * q], acc[0][db][4 * q + 1], acc[0][db][4 * q + 2], acc[0][db][4 * q + 3]});
-      lds_put<f32x2>(stat, f32x2{m_run[0], l_run[0]});
-    }
-    __syncthreads();
-    if (grp > 0) return;
-    float ms[KS], m_all = m_run[0], by[KS];
-    ms[0] = m_run[0];
-    float ls[KS];
-    ls[0] = l_run[0];
-#pragma unroll
-    for (int k = 1; k < KS; ++k) {
-      const f32x2 ml = lds_get<f32x2>(stat + k * NW * 512);
-      ms[k] = ml.x;
-      ls[k] = ml.y;
-      m_all = fmaxf(m_all, ms[k]);
-    }
-    float l_all = 0.f;
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      by[k] = ms[k] > -INFINITY ? fast_exp2(ms[k] - m_all) : 0.f;  // (a group that has seen no key of the row)
-      l_all = fmaf(ls[k], by[k], l_all);
-    }
-    m_run[0] = m_all;
-    l_run[0] = l_all;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f32x4 v = {acc[0][db][4 * q], acc[0][db][4 * q + 1], acc[0][db][4 * q + 2], acc[0][db][4 * q + 3]};
-        v *= by[0];
-#pragma unroll
-        for (int k = 1; k < KS; ++k) v += lds_get<f32x4>(share + k * NW * (NDB * 4096) + (db * 4 + q) * 1024) * by[k];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[0][db][4 * q + t] = v[t];
-      }
   }
 
 #pragma unroll
@@ -1209,25 +1155,24 @@ __device__ __forceinline__ void interval_ends(const AttnParams& p, const BwdSide
 
 // dQ: same tiling as the forward (a workgroup covers 128 rows: BwdSide's padding).
 //   P^T = exp2(S'^T - lse), dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
-template <int D, int NW, int KS = 1>
+template <int D, int NW>
 struct DqSmem {
   // the row-major K and V tiles, 64 keys each; the K^T fragments of the dQ product come
   // out of the K tile through transposing LDS reads
   static constexpr int kTileK = kBN * D * 2;
   static constexpr int kBuf = 2 * kTileK;
-  static constexpr int kDiag = NW * KS * 2 * 32 * D * 2;  // K and V rows of 32 queries per wave (TTT diagonal keys)
-  static constexpr bool kWide = D != 128 && KS == 1;  // attn_bwd_dq_kernel's wide_pass
-  static constexpr int kStages = D == 64 && KS == 1 ? 3 : 2;
-  static constexpr int kTiles = KS * kStages * kBuf > kDiag ? KS * kStages * kBuf : kDiag;
-  static constexpr int kBytes = kTiles + 4 * NW * KS * (int)sizeof(int);
+  static constexpr int kDiag = NW * 2 * 32 * D * 2;  // K and V rows of 32 queries per wave (TTT diagonal keys)
+  static constexpr bool kWide = D != 128;  // attn_bwd_dq_kernel's wide_pass
+  static constexpr int kStages = D == 64 ? 3 : 2;
+  static constexpr int kTiles = kStages * kBuf > kDiag ? kStages * kBuf : kDiag;
+  static constexpr int kBytes = kTiles + 4 * NW * (int)sizeof(int);
 };
 
-template <int D, int NSB, int NW, int KS = 1>
-__global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_dq_kernel(
+template <int D, int NSB, int NW>
+__global__ __launch_bounds__(64 * NW, D > 128 ? 1 : SPX_DQ_MINB) void attn_bwd_dq_kernel(
     AttnParams p, const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     BwdSide sd, uint16_t* __restrict__ dQ, int64_t dq_hs) {
-  static_assert(KS == 1 || (NSB == 1 && D <= 128), "groups of waves: few_workgroups");
-  using SM = DqSmem<D, NW, KS>;
+  using SM = DqSmem<D, NW>;
   constexpr int TB = kBN;
   constexpr int NKK = D / 16;
   constexpr int NDB = D / 32;
@@ -1247,8 +1192,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
   const int m0 = qb * BM;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = KS > 1 ? wave_all % NW : wave_all, grp = KS > 1 ? wave_all / NW : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, col = lane & 31;
   int i[NSB], ic[NSB];
   float lse_i[NSB], delta_i[NSB];
@@ -1258,10 +1202,10 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
     ic[sb] = i[sb] < p.NQ ? i[sb] : p.NQ - 1;
     lse_i[sb] = LSE[(int64_t)h * p.NQ + ic[sb]];
   }
-  if (h == 0 && grp == 0)
+  if (h == 0)
     for (int t = wave; t < BM / 64; t += NW) interval_ends(p, sd, m0 / 64 + t, lane);
   RowBounds<NSB> rb;
-  load_bounds<NSB, NW * KS>(p, ic, wave_all, lane, red, rb);
+  load_bounds<NSB, NW>(p, ic, wave, lane, red, rb);
 
   // the query fragments carry scale * log2(e) (see scale_bf16x8); -lse and -delta of the lane's
   // query sit in all sixteen slots of two blocks that the first MFMA of each product takes as its
@@ -1290,13 +1234,13 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
     }
     delta_i[sb] = half_swap_sum(dot);
     const bool live = i[sb] < p.NQ;
-    if (live && grp == 0) {
+    if (live) {
       uint16_t* qrow_s = sd.qs + ((int64_t)h * p.NQ + i[sb]) * D + g * 8;
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk)
         *reinterpret_cast<u32x4*>(qrow_s + kk * 16) = __builtin_bit_cast(u32x4, qf[sb][kk]);
     }
-    if (g == 0 && grp == 0) {
+    if (g == 0) {
       if (live) sd.delta[(int64_t)h * p.NQ + i[sb]] = delta_i[sb];
       sd.neg[(int64_t)h * sd.NQp + i[sb]] = live ? -lse_i[sb] : 0.f;
       sd.neg[((int64_t)p.Hq + h) * sd.NQp + i[sb]] = live ? -delta_i[sb] : 0.f;
@@ -1321,8 +1265,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
   constexpr int LPK = (TB * RBK / 1024) / NW;
   // (transposing reads touch 4 + 4 rows x 64 bytes: those rows must fall into different 64-byte bank groups)
   auto swz_k = [](int r) { return CKK == 8 ? ((r & 4) | ((r >> 2) & 2) | ((r >> 1) & 1)) : ((r & 3) << 2) | ((r >> 2) & 3); };
-  const uint32_t lds_all = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dq_smem;
-  const uint32_t lds0 = lds_all + grp * (SM::kStages * SM::kBuf);  // this group's tile buffers
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dq_smem;
   const u32x4 kres = make_rsrc(Kh, (uint32_t)((int64_t)p.NKV * RBK));
   const u32x4 vres = make_rsrc(Vh, (uint32_t)((int64_t)p.NKV * RBK));
   auto issue = [&](int n0, int b) __attribute__((always_inline)) {
@@ -1349,16 +1292,15 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
   auto run_pass = [&](const int (&aa)[NSB], const int (&bb)[NSB], int w_amin, int w_amax,
                       int w_bmin, int w_bmax, int blk_a, int blk_b) {
     if (blk_b <= blk_a) return;
-    const int n_first = (blk_a / TB) * TB;
+    const int n_begin = (blk_a / TB) * TB;
     int buf = 0;
     __syncthreads();  // a previous pass may still be reading either buffer
-    if (KS == 1 || n_first + grp * TB < blk_b) issue(n_first + grp * TB, 0);
-    for (int n_turn = n_first; n_turn < blk_b; n_turn += KS * TB) {  // (as many turns for every group, see the forward)
-      const int n0 = n_turn + grp * TB;
+    issue(n_begin, 0);
+    for (int n0 = n_begin; n0 < blk_b; n0 += TB) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (n0 + KS * TB < blk_b) issue(n0 + KS * TB, buf ^ 1);
-      const uint8_t* const tile = dq_smem + grp * (SM::kStages * SM::kBuf) + buf * SM::kBuf;
+      if (n0 + TB < blk_b) issue(n0 + TB, buf ^ 1);
+      const uint8_t* const tile = dq_smem + buf * SM::kBuf;
       buf ^= 1;
       if (n0 >= w_bmax || n0 + TB <= w_amin) continue;
 
@@ -1447,8 +1389,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
   // 64 moves between the register files per half tile), 2520 like this (78 % at 1.6 GHz: at the power limit).  32 heads of 64:
   // 512 rows 15.7 and 14.7, 4096 125 and 114, 8192 under a window of 2048 209 and 196.  At head_dim 128 this needs more
   // registers than two waves of a SIMD have, and with one wave a call of more than one workgroup per compute unit loses:
-  // 4096 rows of 32 heads 227 and 233, 8192 of 64 1370 and 1424 (1024 of 32: 32.2 and 27.8).  Nor do two groups of waves (KS) take
-  // it: the other form and this one, head_dim 64, 128 rows of 32 heads 7.6 and 8.1, 512 12.5 and 12.8, 1024 19.6 and 18.8.
+  // 4096 rows of 32 heads 227 and 233, 8192 of 64 1370 and 1424 (1024 of 32: 32.2 and 27.8).
   // (auto: head sizes that do not call it get no body of it, whose fragments their arrays have no room for)
   auto wide_pass = [&](auto a_i, int b_i, int w_amin, int w_amax, int w_bmin, int w_bmax, int blk_a, int blk_b) {
     static_assert(NSB == 1, "one 32-row block per wave");
@@ -1635,7 +1576,7 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
     static_assert(NSB == 1, "one 32-row block per wave");
     constexpr int XCK = RBK / 16, XRL = 1024 / RBK, XNL = 32 / XRL;
     __syncthreads();  // every wave is done with the tile buffers
-    const uint32_t xk = lds_all + wave_all * (2 * 32 * RBK), xv = xk + 32 * RBK;
+    const uint32_t xk = lds0 + wave * (2 * 32 * RBK), xv = xk + 32 * RBK;
     const int64_t kv_bytes = (int64_t)(p.n_extra + 1) * p.T * RBK;
     const u32x4 xkres = make_rsrc(Kh, (uint32_t)kv_bytes);
     const u32x4 xvres = make_rsrc(Vh, (uint32_t)kv_bytes);
@@ -1651,10 +1592,10 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
 #pragma unroll
       for (int n = 0; n < XNL; ++n) load_to_lds16<0>(res, dst + n * 1024, goff[n], soff);
     };
-    const uint8_t* const xkp = dq_smem + wave_all * (2 * 32 * RBK);
+    const uint8_t* const xkp = dq_smem + wave * (2 * 32 * RBK);
     const uint8_t* const xvp = xkp + 32 * RBK;
     const int xrow = col * RBK, xsw = col & (XCK - 1);
-    for (int j = 1 + grp; j <= p.n_extra; j += KS) {
+    for (int j = 1; j <= p.n_extra; ++j) {
       issue_x(xkres, xk, j);
       issue_x(xvres, xv, j);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1680,31 +1621,6 @@ __global__ __launch_bounds__(64 * NW * KS, D > 128 ? 1 : SPX_DQ_MINB) void attn_
         }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // rows read before the next step overwrites them
     }
-  }
-
-  if constexpr (KS > 1) {  // the groups' sums meet in the first, each through its wave's share of the tile buffers
-    __syncthreads();
-    const uint32_t share = lds_all + wave_all * (NDB * 4096) + lane * 16;
-    static_assert(NW * KS * NDB * 4096 <= SM::kTiles, "32 rows x D sums a wave");
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 v = {acc[0][db][4 * q], acc[0][db][4 * q + 1], acc[0][db][4 * q + 2], acc[0][db][4 * q + 3]};
-        if (grp > 0) lds_put<f32x4>(share + (db * 4 + q) * 1024, v);
-      }
-    __syncthreads();
-    if (grp > 0) return;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int k = 1; k < KS; ++k) {
-          const f32x4 v = lds_get<f32x4>(share + k * NW * (NDB * 4096) + (db * 4 + q) * 1024);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) acc[0][db][4 * q + t] += v[t];
-        }
   }
 
 #pragma unroll
@@ -1919,18 +1835,6 @@ static DkvPlan dkv_plan(int64_t NQ, int64_t NKV, int Hq, int Hkv, int D) {
   return pl;
 }
 
-// Forward and dQ of calls whose workgroups of 128 rows would hardly fill the chip: workgroups of 64 rows, whose four waves are two
-// groups that take every other key tile and add what they have at the end.  Such a call is one round that lasts as long as its
-// longest chain of tiles (0.9 us each at head_dim 64, one wave a SIMD); half as many rows make twice as many workgroups, and two
-// groups halve the chain.  32 heads, workgroups of 128 rows / so, us, forward and dQ: head_dim 64 128 rows 7.3 / 6.6 and 9.2 / 7.6,
-// 512 12.8 / 10.0 and 14.6 / 12.5, 1024 20.3 / 15.7 and 20.8 / 19.6, 1024 in three documents 15.8 / 13.6 and 17.0 / 16.8, but 1300 in four
-// 15.5 / 16.2 and 18.0 / 21.5; head_dim 128 (one workgroup a compute unit: 128 KB) 128 rows 9.1 / 8.3 and 12.5 / 10.9, 512 18.0 / 14.2 and
-// 21.4 / 16.3, in four documents 13.8 / 11.4 and 16.7 / 13.6, but 700 in four 18.7 / 20.6 and 21.8 / 24.6.  Up to one tile of keys there is
-// nothing to share: 64 rows 5.9 / 6.5, 6.9 / 7.8.  (Four groups over 64 rows 512 10.5, 1024 21.1; two over 128 rows 12.1, 18.1.)
-static bool few_workgroups(const AttnParams& p, int D) {
-  return p.NKV > kBN && (int64_t)((p.NQ + kBM - 1) / kBM) * p.Hq <= (D == 64 ? 256 : 128);
-}
-
 // Forward calls of little work take V^T from transposing reads, larger ones from a copy: the copy pays above about 60 us of
 // products at head_dim <= 128 and 1000 us at 256 (at 800 TFLOP/s of a causal mask).  Measured, copy + kernel against
 // transposing reads: 512 rows, 32 heads of 64 16.9 / 13.4 us, 2048 of 128 57.7 / 58.3, 4096 of 128 145 / 147; 600 rows of
@@ -1952,20 +1856,20 @@ static int64_t bwd_workspace_bytes(int64_t NQ, int64_t NKV, int Hq, int Hkv, int
   return b;
 }
 
-template <int D, bool TR, int NW = kFwdNW, int KS = 1>
+template <int D, bool TR>
 static int fwd_lds(const char* fn) {
   static std::atomic<uint64_t> lds_set;  // per instantiation, one bit per device
-  return ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, NW, TR, KS>),
-                            FwdSmem<D, NW, KS>::kBytes, lds_set, fn);
+  return ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>),
+                            FwdSmem<D, kFwdNW>::kBytes, lds_set, fn);
 }
 
-template <int D, bool TR, int NW = kFwdNW, int KS = 1>
+template <int D, bool TR>
 static int launch_fwd_as(AttnParams p, const uint16_t* vt, uint16_t* O, float* lse, hipStream_t st, const char* fn) {
-  constexpr int BM = 32 * kFwdNSB * NW;
+  constexpr int BM = 32 * kFwdNSB * kFwdNW;
   const int n_qb = (p.NQ + BM - 1) / BM;
-  constexpr int smem = FwdSmem<D, NW, KS>::kBytes;
-  if (int rc = fwd_lds<D, TR, NW, KS>(fn)) return rc;
-  hipLaunchKernelGGL((attn_fwd_kernel<D, kFwdNSB, NW, TR, KS>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * NW * KS), smem,
+  constexpr int smem = FwdSmem<D, kFwdNW>::kBytes;
+  if (int rc = fwd_lds<D, TR>(fn)) return rc;
+  hipLaunchKernelGGL((attn_fwd_kernel<D, kFwdNSB, kFwdNW, TR>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kFwdNW), smem,
                      st, p, vt, O, lse);
   return check_launch(fn);
 }
@@ -1977,31 +1881,13 @@ static int launch_fwd(AttnParams p, void* workspace, uint16_t* O, float* lse, hi
     last_error() = std::string(fn) + ": keys of one head must span less than 2 GiB";
     return SPX_ERR_ARG;
   }
-  if (!workspace || fwd_tr(p.NQ, p.NKV, p.Hq, D)) {
-    if constexpr (D <= 128)
-      if (few_workgroups(p, D)) return launch_fwd_as<D, true, 2, 2>(p, nullptr, O, lse, st, fn);
-    return launch_fwd_as<D, true>(p, nullptr, O, lse, st, fn);
-  }
+  if (!workspace || fwd_tr(p.NQ, p.NKV, p.Hq, D)) return launch_fwd_as<D, true>(p, nullptr, O, lse, st, fn);
   uint16_t* vt = reinterpret_cast<uint16_t*>(workspace);
   dim3 tgrid((unsigned)(p.NKVp / 64), (unsigned)((D + 63) / 64), (unsigned)p.Hkv);
   hipLaunchKernelGGL(transpose_bf16_kernel, tgrid, dim3(64), 0, st, p.V, p.v_hs, (int64_t)D, p.NKV, D,
                      vt, (int64_t)D * p.NKVp, D > 128 ? (int64_t)32 : (int64_t)p.NKVp,
                      D > 128 ? (int64_t)32 * D : (int64_t)32);
   return launch_fwd_as<D, false>(p, vt, O, lse, st, fn);
-}
-
-template <int D, int NW, int KS>
-static int launch_dq(const AttnParams& p, const uint16_t* Op, const uint16_t* dOp, const float* lse, const BwdSide& side,
-                     uint16_t* dQp, int64_t dq_hs, hipStream_t st, const char* fn) {
-  constexpr int BM = 32 * kDqNSB * NW, smem = DqSmem<D, NW, KS>::kBytes;
-  static_assert(BM % 64 == 0 && 128 % BM == 0, "BwdSide: whole tiles of 64 rows, rounded up to 128");
-  const int n_qb = (p.NQ + BM - 1) / BM;
-  static std::atomic<uint64_t> lds_set;  // per instantiation, one bit per device
-  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, kDqNSB, NW, KS>), smem, lds_set, fn))
-    return rc;
-  hipLaunchKernelGGL((attn_bwd_dq_kernel<D, kDqNSB, NW, KS>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * NW * KS), smem, st, p, Op,
-                     dOp, lse, side, dQp, dq_hs);
-  return check_launch(fn);
 }
 
 template <int D, bool WHOLE>
@@ -2062,16 +1948,21 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
   }
   const BwdSide side = {NQp, qs, delta, neg, tb, mrows};
 
+  constexpr int BM = 32 * kDqNSB * kDqNW;
+  static_assert(BM == 128, "the rows of BwdSide are rounded up to a workgroup's");
+  const int n_qb = (p.NQ + BM - 1) / BM;
   {
+    constexpr int dq_smem = DqSmem<D, kDqNW>::kBytes;
     if ((int64_t)p.NKVp * D * 2 >= (1ll << 31)) {
       last_error() = std::string(fn) + ": keys of one head must span less than 2 GiB";
       return SPX_ERR_ARG;
     }
-    constexpr int kFewNW = D <= 128 ? 2 : kDqNW, kFewKS = D <= 128 ? 2 : 1;
-    const bool few = D <= 128 && few_workgroups(p, D);
-    if (int rc = few ? launch_dq<D, kFewNW, kFewKS>(p, Op, dOp, lse, side, dQp, dq_hs, st, fn)
-                     : launch_dq<D, kDqNW, 1>(p, Op, dOp, lse, side, dQp, dq_hs, st, fn))
+    static std::atomic<uint64_t> dq_lds_set;  // per head_dim instantiation, one bit per device
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<D, kDqNSB, kDqNW>), dq_smem,
+                                    dq_lds_set, fn))
       return rc;
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, kDqNSB, kDqNW>), dim3((unsigned)(n_qb * p.Hq)), dim3(64 * kDqNW), dq_smem,
+                       st, p, Op, dOp, lse, side, dQp, dq_hs);
   }
 
   const bool whole = pl.whole(p.Hkv);
@@ -2379,10 +2270,8 @@ extern "C" int spx_ttt_attn_fwd_static(const void* q, int64_t q_head_stride, con
     if (int rc = ttt_attn_fwd_impl(fname, q, q_head_stride, k, k_head_stride, v, v_head_stride, row_lo, T, ttt_step, Hq, Hkv,
                                    D, scaling, out, lse, workspace, stream))
       return rc;
-    // the forms that captured calls take are set up by the first call too, which is made outside capture
-    if (D == 256) return fwd_lds<256, true>(fname);
-    if (int rc = D == 128 ? fwd_lds<128, true>(fname) : fwd_lds<64, true>(fname)) return rc;
-    return D == 128 ? fwd_lds<128, true, 2, 2>(fname) : fwd_lds<64, true, 2, 2>(fname);
+    // the form that captured calls take is set up by the first call too, which is made outside capture
+    return D == 256 ? fwd_lds<256, true>(fname) : D == 128 ? fwd_lds<128, true>(fname) : fwd_lds<64, true>(fname);
   });
 }
 

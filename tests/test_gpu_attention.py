@@ -265,10 +265,33 @@ def test_random_shapes_forward_and_backward(t, hq, hkv, d, docs, window, steps):
     (385, 32, 8, 128, [1, 300, 60], 100, 2), (257, 44, 11, 128, None, None, 3),
     (64, 4, 2, 64, None, None, 3), (65, 4, 2, 64, [64], None, 4), (65, 4, 2, 128, None, None, 2),  # one key tile, and one row more
 ])
-def test_both_sides_of_few_workgroups(t, hq, hkv, d, docs, window, steps):
-    """Calls of few workgroups run on workgroups of two groups of waves over every other key tile each."""
+def test_calls_of_few_workgroups(t, hq, hkv, d, docs, window, steps):
+    """Calls of fewer workgroups than the chip has room for, of as many and of more."""
     test_forward_matches_dense_oracle(t, hq, hkv, d, docs, window, steps)
     test_backward_matches_dense_oracle_autograd(t, hq, hkv, d, docs, window, steps)
+
+
+@pytest.mark.parametrize("t,hq,hkv,d,docs,copies", [
+    (300, 8, 2, 64, [170, 130], 16), (65, 4, 2, 64, None, 80),      # 24 workgroups of 128 rows and 384, 4 and 320
+    (257, 8, 2, 128, None, 8), (130, 4, 1, 128, [60, 70], 20),      # 24 and 192, 8 and 160
+])
+def test_a_heads_results_do_not_depend_on_how_many_heads_a_call_has(t, hq, hkv, d, docs, copies):
+    """Output and dQ of the same heads alone and among copies of them, bit for bit: the probabilities are rounded
+    against one running maximum of all keys in front of them, however few workgroups there are."""
+    from speculators_amd.attention import create_ttt_mask, ttt_attention
+
+    g = torch.Generator().manual_seed(11 * t + d)
+    doc = torch.zeros(t, dtype=torch.long) if docs is None else _docs(t, docs)
+    mask = create_ttt_mask(doc.cuda(), t, None).extended()
+    q, k, v = (torch.randn(1, h, n, d, generator=g).bfloat16().cuda() for h, n in ((hq, t), (hkv, 2 * t), (hkv, 2 * t)))
+    go = torch.randn(1, t, hq, d, generator=g).bfloat16().cuda()
+    got = []
+    for n in (1, copies):
+        qn, kn, vn = (x.repeat(1, n, 1, 1).requires_grad_(True) for x in (q, k, v))
+        out = ttt_attention(qn, kn, vn, mask, d ** -0.5)
+        out.backward(go.repeat(1, 1, n, 1))
+        got.append((out.detach()[:, :, :hq], qn.grad[:, :hq]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
 @pytest.mark.parametrize("t,hq,hkv,d,docs,window,steps", [

@@ -115,6 +115,27 @@ def test_key_blocks_one_by_one(t, hq, hkv, d):
     test_forward_backward_match_dense_oracle(t, hq, hkv, d, [t], sorted(anchors), 16, None, False)
 
 
+@pytest.mark.parametrize("t,d,window,copies", [(1024, 64, 100, 16), (700, 64, None, 16), (512, 128, None, 8)])
+def test_a_heads_results_do_not_depend_on_how_many_heads_a_call_has(t, d, window, copies):
+    """Output and dQ of the same heads of a few blocks alone and among copies of them, bit for bit."""
+    from speculators_amd.attention import create_dflash_mask, dflash_attention
+
+    g = torch.Generator().manual_seed(t + d)
+    hq, hkv, bs = 8, 2, 8
+    anchors = torch.randperm(t - bs - 1, generator=g)[:40].sort().values + 1
+    nq = 40 * bs
+    mask = create_dflash_mask(_docs(t, [t // 3, t - t // 3]).cuda(), t, anchors.cuda(), bs, window, False)
+    q, k, v = (torch.randn(1, h, n, d, generator=g).bfloat16().cuda() for h, n in ((hq, nq), (hkv, t + nq), (hkv, t + nq)))
+    go = torch.randn(1, nq, hq, d, generator=g).bfloat16().cuda()
+    got = []
+    for n in (1, copies):
+        qn, kn, vn = (x.repeat(1, n, 1, 1).requires_grad_(True) for x in (q, k, v))
+        out = dflash_attention(qn, kn, vn, mask, d ** -0.5)
+        out.backward(go.repeat(1, 1, n, 1))
+        got.append((out.detach()[:, :, :hq], qn.grad[:, :hq]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("weighting,sliding,head_dim", [("fixed-exp-decay", False, 64), ("dpace", True, 64),
                                                         ("fixed-exp-decay", True, 96)])
 def test_model_forward_backward_matches_oracle(weighting, sliding, head_dim):
