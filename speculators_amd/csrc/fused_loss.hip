@@ -86,14 +86,15 @@ __device__ __forceinline__ RowStats block_merge(RowStats s, RowStats* part) {
   return wave_merge<DRAFT>(s);
 }
 
-// log2 p - log2 m and log2 q - log2 m of the mean m of two probabilities p and q with the natural logarithms ldp and ltp: the
-// larger one's logarithm cancels, so no term of its size stands in either.  (No expression that the compiler could fuse in one
-// direction and not in the other.)
+// log p - log m and log q - log m of the mean m of two probabilities p and q with the logarithms ldp and ltp: the larger one's
+// logarithm cancels, so no term of its size stands in either.  In natural units: a column at the type's lowest value on one side has
+// a finite difference, and 0 times it is nothing (times log2(e) it would be infinite, and the row not a number).  (No expression that
+// the compiler could fuse in one direction and not in the other.)
 struct MixLogs { float p, q; };
 __device__ __forceinline__ MixLogs mix_logs(float ldp, float ltp) {
-  const float d = (ldp - ltp) * kLog2e;
-  const float w = 1.f - fast_log2(1.f + fast_exp2(-fabsf(d)));
-  return {w + fminf(d, 0.f), w - fmaxf(d, 0.f)};
+  const float d = ldp - ltp;
+  const float w = 1.f - fast_log2(1.f + fast_exp2(-fabsf(d) * kLog2e));
+  return {fmaf(w, kLn2, fminf(d, 0.f)), fmaf(w, kLn2, -fmaxf(d, 0.f))};
 }
 
 __device__ __forceinline__ void store_flag(void* p, int kind, int64_t i, bool v) {
@@ -219,7 +220,7 @@ __device__ __forceinline__ void add_second(float& acc, float& ext, const float (
     const float ldp = x[i] - lse_d, ltp = y[i] - lse_t, a = ldp * kLog2e, b = ltp * kLog2e;
     if (OP == SPX_LOSS_RKL) {
       acc = fmaf(fast_exp2(a), ldp - ltp, acc);
-    } else if (OP == SPX_LOSS_JSD) {  // (in units of log 2)
+    } else if (OP == SPX_LOSS_JSD) {
       const MixLogs l = mix_logs(ldp, ltp);
       acc = fmaf(fast_exp2(a), l.p, acc);
       ext = fmaf(fast_exp2(b), l.q, ext);
@@ -509,7 +510,7 @@ __global__ __launch_bounds__(NT, HELD * sizeof(T) > 16 ? 2 : HELD ? 4 : 1) void 
     }
     acc = block_sum<NT / 64>(acc, red);
     ext = block_sum<NT / 64>(ext, red);
-    if (OP == SPX_LOSS_JSD) { row_loss = 0.5f * kLn2 * (acc + ext); row_extra = acc * kLn2; }
+    if (OP == SPX_LOSS_JSD) { row_loss = 0.5f * (acc + ext); row_extra = acc; }
     else { row_loss = 1.f - acc; row_extra = ext; }
   }
   if (tid == 0) {
@@ -791,7 +792,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     }
     if (has_tv) { sum_v = block_sum<kFgWaves>(sum_v, red); ext_v = block_sum<kFgWaves>(ext_v, red); }
     if (has_rkl) sum_r = block_sum<kFgWaves>(sum_r, red);
-    if (has_jsd) { sum_j = kLn2 * block_sum<kFgWaves>(sum_j, red); ext_j = kLn2 * block_sum<kFgWaves>(ext_j, red); }
+    if (has_jsd) { sum_j = block_sum<kFgWaves>(sum_j, red); ext_j = block_sum<kFgWaves>(ext_j, red); }
   }
   if (tid == 0) {
     const float of[5] = {(KNOWN ? s.at : s.at / s.zt) - lse_t + lse_d, sum_r, 0.5f * (sum_j + ext_j), lse_d - s.xt, 1.f - sum_v};
@@ -832,8 +833,7 @@ __global__ __launch_bounds__(kFgThreads) __attribute__((amdgpu_waves_per_eu(4, 4
       for (int i = 0; i < 8; ++i) {
         const float ldp = x[i] - lse_d, ltp = y[i] - lse_t, dp = fast_exp2(fmaf(x[i], kLog2e, cd));
         if (has_rkl) o[i] = fmaf(tm.w[SPX_LOSS_RKL] * dp, ldp - ltp - sum_r, o[i]);
-        if (has_jsd)
-          o[i] = fmaf(0.5f * tm.w[SPX_LOSS_JSD] * dp, fmaf(mix_logs(ldp, ltp).p, kLn2, -sum_j), o[i]);
+        if (has_jsd) o[i] = fmaf(0.5f * tm.w[SPX_LOSS_JSD] * dp, mix_logs(ldp, ltp).p - sum_j, o[i]);
       }
     }
     if (c == label >> 3) {
@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_bwd_kernel(
         // same expressions as the forward's second walk, so that the
         // q <= p comparison of tv resolves identically in both directions
         const float ldp = x[i] - lse_d, ltp = y[i] - lse_t, dp = fast_exp2(ldp * kLog2e);
-        if (OP == SPX_LOSS_JSD) o[i] = g * 0.5f * dp * fmaf(mix_logs(ldp, ltp).p, kLn2, -ex);
+        if (OP == SPX_LOSS_JSD) o[i] = g * 0.5f * dp * (mix_logs(ldp, ltp).p - ex);
         else o[i] = -g * dp * ((dp <= fast_exp2(ltp * kLog2e) ? 1.f : 0.f) - ex);
       }
     }

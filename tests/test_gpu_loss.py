@@ -110,6 +110,68 @@ def test_two_walks_at_the_edges_of_what_is_held(name, dtype, rows, vocab):
     assert err < (2e-5 if dtype == torch.float32 else 4e-3), err
 
 
+def _closed(name, x, y):
+    """Row losses and the gradient of their sum in float64, where a probability of nothing has no term."""
+    lp, lq = torch.log_softmax(x.double().cpu(), -1), torch.log_softmax(y.double().cpu(), -1)
+    p, q = lp.exp(), lq.exp()
+    if name == "rkl":
+        a = torch.where(p > 0, lp - lq, 0.0)
+        rows = (p * a).sum(-1)
+        return rows, p * (a - rows[..., None])
+    lm = torch.logaddexp(lp, lq) - torch.log(torch.tensor(2.0, dtype=torch.float64))
+    a, b = torch.where(p > 0, lp - lm, 0.0), torch.where(q > 0, lq - lm, 0.0)
+    ext = (p * a).sum(-1)
+    return 0.5 * (ext + (q * b).sum(-1)), 0.5 * p * (a - ext[..., None])
+
+
+def _ruled_out(rows, vocab, dtype, side, value):
+    g = torch.Generator().manual_seed(rows + vocab)
+    x, y = (torch.randn(1, rows, vocab, generator=g) * 2 for _ in range(2))
+    out = torch.rand(vocab, generator=g) < 0.5
+    value = max(value, torch.finfo(dtype).min)
+    if side != "target":
+        x[..., out] = value
+    if side != "draft":
+        y[..., out.roll(1) if side == "both" else out] = value
+    return x.to(dtype), y.to(dtype)
+
+
+# one row a workgroup with the pair held, more threads and fewer, the streaming walk, unaligned rows
+LOWEST = [(3, 4096), (300, 4096), (600, 4096), (3, 33000), (3, 1001)]
+
+
+@pytest.mark.parametrize("side", ["draft", "target", "both"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,vocab", LOWEST)
+@pytest.mark.parametrize("value", [-1e39, -2.4e38, -1e9])
+def test_jsd_where_columns_are_ruled_out(rows, vocab, dtype, side, value):
+    """Half of the columns at the type's lowest value (or above 2^128 / log2(e), or at a usual mask's): they have no term on
+    their side, and the loss stays within log 2."""
+    from speculators_amd import losses as L
+
+    x, y = _ruled_out(rows, vocab, dtype, side, value)
+    xg = x.cuda().requires_grad_(True)
+    out = L.resolve_loss_config("jsd")["jsd"][0](xg, y.cuda())
+    (grad,) = torch.autograd.grad(out, xg, torch.ones_like(out))
+    want, want_grad = _closed("jsd", x, y)
+    torch.testing.assert_close(out.double().cpu(), want, atol=1e-6, rtol=1e-5)
+    assert (grad.double().cpu() - want_grad).norm() <= (2e-5 if dtype == torch.float32 else 4e-3) * want_grad.norm()
+
+
+@pytest.mark.parametrize("rows", [5, 300])
+def test_gathered_jsd_where_target_columns_are_ruled_out(rows):
+    from speculators_amd import losses as L
+
+    for dtype in (torch.float32, torch.bfloat16):
+        x, y = _ruled_out(rows, 2048, dtype, "target", -1e39)
+        full = torch.zeros(rows, 4096, dtype=dtype)
+        full[:, ::2] = y[0]
+        step = L.StepPass(d2t=torch.arange(2048, device="cuda"), mask=None, prev=None,
+                          counts=torch.zeros(3, device="cuda", dtype=torch.int32))
+        loss = L.fused_loss_forward(L.OP_JSD, x[0].cuda(), full.cuda(), None, step)[0]
+        torch.testing.assert_close(loss.double().cpu(), _closed("jsd", x, y)[0][0], atol=1e-6, rtol=1e-5)
+
+
 def test_reverse_kl_of_rows_a_constant_apart():
     """Rows that differ by little but a constant of 30, whose loss is a difference of 1e-4 beside terms of 30; and columns that
     one side or both rule out (-inf), where it is infinite or not a number as the sum of its terms is."""

@@ -80,6 +80,42 @@ def test_terms_in_one_row_pass(spec, vocab):
     assert (dx[0].double().cpu() - ref).abs().max().item() <= 2 ** -6 * ref.abs().max().item()
 
 
+@pytest.mark.parametrize("side", ["draft", "target", "both"])
+def test_terms_where_columns_are_ruled_out(side):
+    """jsd with columns at the type's lowest value: in the target, or in the draft by a head's row."""
+    vocab = 4104
+    x, w, y, mask = _inputs(33, vocab, seed=2)
+    lowest = torch.finfo(torch.bfloat16).min
+    if side != "target":
+        x.data[..., 0] = 1.0
+        w[::3], w[::3, 0] = 0.0, lowest
+    if side != "draft":
+        y[..., 1::3] = lowest
+        if side == "both":
+            y[..., ::6] = lowest
+    total, _, dx, heads, _ = _steps("jsd", x, w, y, mask, 2)
+    logits = heads[0].logits.detach().double().cpu()[0]
+    assert side == "target" or bool((logits[:, ::3] < -3e38).all())
+    want, dl = 0.0, torch.zeros_like(logits)
+    for k in range(2):
+        n = 33 - k
+        lp, lt = logits[:n].log_softmax(-1), y.double().cpu()[0, k:].log_softmax(-1)
+        lm = torch.logaddexp(lp, lt) - torch.tensor(2.0).double().log()
+        p, t, mk = lp.exp(), lt.exp(), mask.double().cpu()[0, k:]
+        a, b = torch.where(p > 0, lp - lm, 0.0), torch.where(t > 0, lt - lm, 0.0)
+        wt = 0.8 ** k * mk / (mk.sum() + 1e-5)
+        ext = (p * a).sum(-1)
+        want = want + (wt * 0.5 * (ext + (t * b).sum(-1))).sum()
+        dl[:n] += 3.0 * 0.5 * wt[:, None] * p * (a - ext[:, None])
+    assert abs(total.item() - want.item()) <= 2e-5 * max(abs(want.item()), 1.0)
+    keep = torch.ones(vocab, dtype=torch.bool)
+    if side != "target":
+        keep[::3] = False
+        assert not bool(dl[:, ::3].any())
+    ref = dl[:, keep] @ w.double().cpu()[keep]
+    assert (dx[0].double().cpu() - ref).abs().max().item() <= 2 ** -6 * ref.abs().max().item()
+
+
 @pytest.mark.parametrize("spec", TERMS)
 def test_terms_count_and_chain_like_the_streaming_pass(spec, monkeypatch):
     got = []
