@@ -17,7 +17,7 @@ namespace spx {
 // ---- running statistics ----------------------------------------------------
 struct RowStats {
   float md, zd;        // draft: running max (base-2 scaled) and sum of 2^(x' - md)
-  float mt, zt, at;    // target: same, and sum of 2^(y' - mt) * (y - x); rkl: of 2^(x' - md) * ((x - bd) - (y - bt))
+  float mt, zt, at;    // target: same, and sum of 2^(y' - mt) * (y - x); rkl: of 2^(x' - md) * ((x - bd) - (y - bt)) * kRklUnit
   float bd; int id;    // draft arg-max value / first index
   float bt; int it; float xt;  // target arg-max value / first index / draft logit there
 };
@@ -25,8 +25,13 @@ struct RowStats {
 // rkl walks a row once: its sum of 2^(x' - md) * ((x - bd) - (y - bt)) is kept beside the soft-max's, relative to the largest
 // values so far (us, read twice / once: bf16 64 x 32000 16.8 / 11.4, 333 22.9 / 18.0, 3000 114 / 80, 1024 x 128256 158 / 98; fp32 333 x
 // 32000 34.0 / 22.9, 1024 x 128256 312 / 185; against float64 its losses are off by 1e-7 in the place of 7e-7, its gradients by 5e-7 in
-// the place of 1e-6).  Here: that sum after the draft's largest value has risen by dx and the target's by dy
-__device__ __forceinline__ float off_by(float at, float z, float dy, float dx) { return z == 0.f ? at : fmaf(z, dy - dx, at); }
+// the place of 1e-6).  It is kept in units of 2^32, exactly: there are up to as many terms as columns, each as large as the type has
+// values where the target rules columns out that the draft gives weight, and only their mean has to be a number.
+constexpr float kRklUnit = 0x1p-32f;
+// that sum after the draft's largest value has risen by dx and the target's by dy
+__device__ __forceinline__ float off_by(float at, float z, float dy, float dx) {
+  return z == 0.f ? at : fmaf(z * kRklUnit, dy - dx, at);
+}
 // A wave's statistics in every lane of it.  The largest value and its first index come first, then every sum is scaled once.
 // (A tree of pairwise merges, ten shuffles a level and two exponentials a sum, and a walk over the waves' results behind it took
 // 2 us of a row: 64 rows of 32000 bf16, kl 13.4 -> 10.0 us, 333 rows 17.9 -> 16.4.)
@@ -183,7 +188,7 @@ __device__ __forceinline__ void add_chunk(RowStats& s, const float (&x)[8], cons
     for (int i = 0; i < 8; ++i) {
       const float e = fast_exp2(fmaf(x[i], kLog2e, -mn));
       z += e;
-      if (OP == SPX_LOSS_RKL) a = fmaf(e, (x[i] - mx) - (y[i] - my), a);
+      if (OP == SPX_LOSS_RKL) a = fmaf(e, fmaf(x[i], kRklUnit, -mx * kRklUnit) - fmaf(y[i], kRklUnit, -my * kRklUnit), a);
     }
     s.zd = z; s.md = mn;
     if (OP == SPX_LOSS_RKL) s.at = a;
@@ -464,7 +469,7 @@ __global__ __launch_bounds__(NT, HELD * sizeof(T) > 16 ? 2 : HELD ? 4 : 1) void 
     // the mean of x - y under the draft's probabilities, less the log-sum-exps' difference, both counted from the rows' largest
     // values: for the loss what lies between those cancels (but for the rounding of md and mt), for the backward it is formed from
     // what is stored and subtracted there, too (rows that are nearly equal, or but for a constant, keep their digits)
-    const float bd = fmaxf(s.bd, kNegBig), bt = fmaxf(s.bt, kNegBig), mean = s.at / s.zd;
+    const float bd = fmaxf(s.bd, kNegBig), bt = fmaxf(s.bt, kNegBig), mean = s.at / s.zd * (1.f / kRklUnit);
     row_loss = mean - (fast_log2(s.zd / s.zt) - (fmaf(bd, kLog2e, -s.md) - fmaf(bt, kLog2e, -s.mt))) * kLn2;
     row_extra = mean + ((bd - lse_d) - (bt - lse_t));
   } else {

@@ -158,8 +158,30 @@ def test_jsd_where_columns_are_ruled_out(rows, vocab, dtype, side, value):
     assert (grad.double().cpu() - want_grad).norm() <= (2e-5 if dtype == torch.float32 else 4e-3) * want_grad.norm()
 
 
+@pytest.mark.parametrize("side", ["draft", "target", "both"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,vocab", LOWEST)
+@pytest.mark.parametrize("value", [-1e39, -1e30, -1e9])
+def test_rkl_where_columns_are_ruled_out(rows, vocab, dtype, side, value):
+    """Columns that the target rules out and the draft gives weight: the loss is that weight times the value, though the terms
+    before the division by the soft-max's sum are too large for the type.  (fp32 sums of terms of one sign: 1e-5.  A gradient's
+    rounding is that of the values' differences, 2^-23 of the value times the probability.  Where the draft rules columns out, too,
+    their logarithm at the type's lowest value less such a loss is none of the type, and the row has no gradient.)"""
+    from speculators_amd import losses as L
+
+    x, y = _ruled_out(rows, vocab, dtype, side, value)
+    xg = x.cuda().requires_grad_(True)
+    out = L.resolve_loss_config("rkl")["rkl"][0](xg, y.cuda())
+    (grad,) = torch.autograd.grad(out, xg, torch.ones_like(out))
+    want, want_grad = _closed("rkl", x, y)
+    torch.testing.assert_close(out.double().cpu(), want, atol=1e-6, rtol=1e-5)
+    if side != "both" or value > -1e38:
+        assert (grad.double().cpu() - want_grad).norm() <= (2e-5 if dtype == torch.float32 else 4e-3) * want_grad.norm()
+
+
 @pytest.mark.parametrize("rows", [5, 300])
-def test_gathered_jsd_where_target_columns_are_ruled_out(rows):
+@pytest.mark.parametrize("name", ["jsd", "rkl"])
+def test_gathered_losses_where_target_columns_are_ruled_out(rows, name):
     from speculators_amd import losses as L
 
     for dtype in (torch.float32, torch.bfloat16):
@@ -168,8 +190,8 @@ def test_gathered_jsd_where_target_columns_are_ruled_out(rows):
         full[:, ::2] = y[0]
         step = L.StepPass(d2t=torch.arange(2048, device="cuda"), mask=None, prev=None,
                           counts=torch.zeros(3, device="cuda", dtype=torch.int32))
-        loss = L.fused_loss_forward(L.OP_JSD, x[0].cuda(), full.cuda(), None, step)[0]
-        torch.testing.assert_close(loss.double().cpu(), _closed("jsd", x, y)[0][0], atol=1e-6, rtol=1e-5)
+        loss = L.fused_loss_forward(L.PRIMITIVE_OP[name], x[0].cuda(), full.cuda(), None, step)[0]
+        torch.testing.assert_close(loss.double().cpu(), _closed(name, x, y)[0][0], atol=1e-6, rtol=1e-5)
 
 
 def test_reverse_kl_of_rows_a_constant_apart():
