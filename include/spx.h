@@ -769,8 +769,8 @@ int spx_gemm_bf16_pair(int form, const void* a, int64_t lda, const void* b, cons
                        int64_t M, int64_t N, int64_t K, int32_t max_parts, void* workspace, int64_t workspace_bytes,
                        int32_t* parts, void* stream);
 
-/* The first product of a gated MLP: act = silu(a gate^T) (a up^T) [M, F] (rounded as spx_swiglu_rows_fwd does, 1 / (1 + e^-x) within
- * two units of fp32), gate and up [F, K], ldb apart; gu (or NULL): [M, 2 F], the two results.  spx_gemm_gated_takes: the sizes where it
+/* The first product of a gated MLP: act = silu(a gate^T) (a up^T) [M, F] (spx_swiglu_rows_fwd of the two results as they are rounded, its
+ * bits but for gates below -87, where 1 / (1 + e^-x) is no normal number), gate and up [F, K], ldb apart; gu (or NULL): [M, 2 F], the two results.  spx_gemm_gated_takes: the sizes where it
  * takes the place of the product and that pass; others run too, where F is a multiple of 256 and K of 64, at least 192.  A last round
  * is cut into up to max_parts as spx_gemm_bf16_nt_tail has it where the workspace (or NULL) is as large as that asks for. */
 int spx_gemm_gated_takes(int64_t M, int64_t F, int64_t K, int64_t ldb, int32_t max_parts);

@@ -21,12 +21,14 @@ namespace spx {
 constexpr int kSlowRow = kTN * 2;  // SLOW: bytes of a row of a slab of B
 static_assert(kTK * kSlowRow == kBBytes && kTK / 2 / kNW == kLB, "a slab is as large either way");
 
-// silu(g) u of eight pairs, as swiglu_fwd_kernel rounds it; 1 / (1 + e^-g) by the reciprocal instruction, of a quarter of the sum
-// (the reciprocal of a sum above 2^126 would be flushed to zero).
+// silu(g) u of eight pairs, the bits of swiglu_fwd_kernel.  1 / (1 + e^-g) by the reciprocal instruction and one step of Newton's, whose
+// residue is exact, in the place of a division's ten instructions; of a quarter of the sum (the reciprocal of a sum above 2^126 would
+// be flushed to zero), and of an infinite sum it is nothing, with or without the step.
 __device__ __forceinline__ u32x4 swiglu8(u32x4 g, u32x4 u) {
   auto silu = [](float gv) __attribute__((always_inline)) {
     const float quarter = gv * 0.25f, e = fast_exp2(quarter * (-4.f * 1.44269504f));
-    return quarter * __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f));
+    const float sum = fmaf(e, 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(sum);
+    return quarter * fmaf(r, fmaf(-fminf(sum, 0x1p127f), r, 1.f), r);
   };
   u32x4 o;
 #pragma unroll
@@ -49,7 +51,7 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 // cost all products of that form 0.5 - 1.4 %.)
 // GATE: a gated MLP's first product.  B is the gate's weight, B2 that of the up projection, `half` rows each (a multiple of 256); a
 // tile is 128 columns of each, in every wave 64 and the same 64, so that a lane holds what belongs together: `act` =
-// swiglu_of(gate, up) from the two results as they are rounded (bf16 [M, half], ld_act apart), which leave too where GATE is 2 (in
+// swiglu8(gate, up) from the two results as they are rounded (bf16 [M, half], ld_act apart), which leave too where GATE is 2 (in
 // C, the gate's columns and behind them the up projection's).  A cut tile's parts lie as its columns do.  Product and SwiGLU launch / this, us (of the launch, bound by
 // its traffic, the activation's arithmetic remains, 2.4 us a round of tiles that nothing runs beside): 1999 x 2048 -> 2 x 8192 without
 // the two results 118 / 101, 888 rows with them 60.6 / 54.2, 4096 x 4096 -> 2 x 14336 703 (the product the library's) / 665, 8192 rows 1368 / 1327, 3001
