@@ -1908,9 +1908,12 @@ static int launch_bwd(AttnParams p, const uint16_t* Op, const uint16_t* dOp, con
                       int64_t dv_hs, void* workspace, hipStream_t st, const char* fn, int accumulate = 0) {
   const int NQp = (int)round_up(p.NQ, 128);
   DkvPlan pl = dkv_plan(p.NQ, p.NKV, p.Hq, p.Hkv, D);
-  // Rows that see a context and a block of their own: pairs of key blocks are not equally long then (8192 + 8192 keys, 8192 rows of
-  // 32 heads of 128: 651 us in pairs, 618 without)
-  if (p.a2 && pl.paired) {
+  // Rows that see a context and a block of their own: pairs of key blocks are not equally long then.  Single blocks took 0.91 of the
+  // time over 105 calls of 1248 to 8192 rows, in one to six documents and under a window, 1.09 at the most (8192 + 8192 keys, 8192 rows
+  // of 32 heads of 128 under a window of 2048 568 -> 543 us, 2048 + 4096 in six documents 174 -> 111).  Where the pairs of few rows fit
+  // in one round, the starts of a second one weigh more: 512 to 1248 rows 1.05 over 33 calls (1024 + 1024 keys, 32 heads of 128
+  // 55 -> 69 us, 64 heads 86 -> 105), but 1488 and 1776 rows 0.93; at head_dim 256 512 to 1024 rows 1.01, 1248 0.89.
+  if (p.a2 && pl.paired && (pl.n_k * pl.n_hu > 256 * (D == 64 ? 2 : 1) || p.NQ > (D > 128 ? 1024 : 1280))) {
     pl.paired = 0;
     pl.n_k = pl.n_kb;
   }

@@ -108,11 +108,17 @@ def test_random_shapes(t, hq, hkv, d, docs, anchors, bs, window, ncf):
     test_forward_backward_match_dense_oracle(t, hq, hkv, d, docs, anchors, bs, window, ncf)
 
 
-# (long enough that a causal mask would have the key blocks in pairs; one and two of two and of eight heads a workgroup)
+# (long enough that the key blocks are in pairs; one and two of two and of eight heads a workgroup)
 @pytest.mark.parametrize("t,hq,hkv,d", [(200, 64, 64, 64), (65, 64, 4, 64), (300, 128, 64, 128), (200, 128, 16, 64)])
-def test_key_blocks_one_by_one(t, hq, hkv, d):
+def test_key_blocks_in_pairs(t, hq, hkv, d):
     anchors = [(7 * i) % t for i in range(24 if d == 128 else 32 if t > 65 else 48)]
     test_forward_backward_match_dense_oracle(t, hq, hkv, d, [t], sorted(anchors), 16, None, False)
+
+
+# (more rows than key blocks are in pairs for; partial results of one head, and a workgroup with all heads of its K/V head)
+@pytest.mark.parametrize("t,hq,hkv,d,n", [(200, 32, 8, 64, 81), (200, 32, 32, 64, 81), (700, 24, 3, 128, 81), (700, 16, 16, 256, 66)])
+def test_key_blocks_one_by_one(t, hq, hkv, d, n):
+    test_forward_backward_match_dense_oracle(t, hq, hkv, d, [t // 3, t - t // 3], sorted((7 * i) % t for i in range(n)), 16, None, False)
 
 
 @pytest.mark.parametrize("t,d,window,copies", [(1024, 64, 100, 16), (700, 64, None, 16), (512, 128, None, 8)])
