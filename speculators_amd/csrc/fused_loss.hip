@@ -1929,19 +1929,26 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // Threads per row: enough that few rows fill the chip (2048 threads per compute unit), not so many that a compute unit holds
 // one row only and waits between them.  It depends on the call's sizes alone: the gathering form of a call adds in the same order
-// and gives the same bits, except that above 64 rows its KL / CE form stays with the pipelined kernel of 256 threads.
+// and gives the same bits, except that above 64 rows its KL / CE form stays with the pipelined kernel of 256 threads, and above 256
+// its fp32 form of jsd and tv with 512 where the plain one has 1024.
 // Measured with 256 threads, a load at a time -> these and one wave's sums by lane moves (us), bf16: KL 64 rows of 128256 76 -> 24,
 // 333 rows of 128256 92 -> 45, of 32000 27 -> 17, 1024 of 32000 33 -> 30; backward (columns over several workgroups) 64 rows of
 // 128256 66 -> 7.
 static int threads_per_row(int64_t rows) { return rows <= 256 ? 1024 : rows <= 512 ? 512 : kLossThreads; }
-// jsd and tv walk a row twice.  Up to 32768 columns the pair stays in a workgroup's registers between the walks: 512 threads a row,
-// two rows a compute unit (bf16), or 1024 and one (fp32, and where there are no more rows than compute units).  Read twice /
-// held, us: jsd bf16 64 x 32000 21.6 / 15.6, 333 32.1 / 28.2, 1024 58.6 / 52.0, 3000 139 / 134 and its backward, which then finds
-// more of the rows in the cache, 113 / 94; tv 3000 119 / 111 and 112 / 88; fp32 jsd 333 40.0 / 36.9, 3000 221 / 206, tv 212 / 192.
+// jsd and tv walk a row twice.  Of some columns on, up to 32768, the pair stays in a workgroup's registers between the walks: 512 threads
+// a row, two rows a compute unit (bf16), or 1024 and one (fp32, and where there are no more rows than compute units).  256 threads that
+// read twice / held, forward + backward, us: jsd bf16 3000 rows of 32000 242 / 231, of 24000 179 / 177, of 16000 125 / 125 (1024 rows
+// 50.3 / 46.8), of 12000 98 / 103; tv 236 / 200, 174 / 156, 121 / 112, 91 / 93; fp32 jsd 453 / 438, 344 / 337, 231 / 243, 169 / 187, tv
+// 448 / 418, 338 / 321, 227 / 230, 166 / 178; forward alone, 3000 rows of 1000 18 / 27 (bf16), 18 / 59 (fp32).  Rows that do not begin
+// at 16 bytes, and the gathering form, have nothing to hold, but the same threads (256 / so, forward: bf16 3000 rows of 32003 485 / 368,
+// gathered 1024 of 32000 154 / 149; gathered fp32 253 with 1024 threads, 247 with 256, 238 with 512).
 static bool walked_twice(int op) { return op == SPX_LOSS_JSD || op == SPX_LOSS_TV; }
-constexpr int64_t kHeldVocab = 32768 + 7;  // (columns behind the last whole chunk are read again)
-static int threads_per_row(int64_t rows, int64_t vocab, int op, bool wide) {
-  return walked_twice(op) && vocab <= kHeldVocab ? (rows <= 256 || wide ? 1024 : 512) : threads_per_row(rows);
+static bool held_vocab(int64_t vocab, bool wide) {
+  return vocab > (wide ? 18432 : 14336) && vocab <= 32768 + 7;  // (columns behind the last whole chunk are read again)
+}
+static int threads_per_row(int64_t rows, int64_t vocab, int op, bool wide, bool gather) {
+  if (!walked_twice(op) || !held_vocab(vocab, wide)) return threads_per_row(rows);
+  return rows <= 256 || (wide && !gather) ? 1024 : 512;
 }
 
 // Rows that the 256 MB cache can hold a good part of are left in it for the backward (forward + backward past the caches / through
@@ -1964,15 +1971,16 @@ static int launch_fwd(const char* fname, int op, const T* lg, int64_t ldl, const
                                       lds, lds_set, fname))                                                        \
         return rc;                                                                                                 \
     }                                                                                                              \
-    constexpr bool held = VEC && !KNOWN && !GATHER && NT >= 512 && (OPV == SPX_LOSS_JSD || OPV == SPX_LOSS_TV);     \
-    if (held && vocab <= kHeldVocab)                                                                               \
+    constexpr bool held = VEC && !KNOWN && !GATHER && (NT == 1024 || (NT == 512 && sizeof(T) == 2)) &&              \
+                          (OPV == SPX_LOSS_JSD || OPV == SPX_LOSS_TV);                                             \
+    if (held && held_vocab(vocab, sizeof(T) == 4))                                                                 \
       hipLaunchKernelGGL((loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER, NT, held ? 4096 / NT : 0>), grid, block, lds, \
                          st, lg, ldl, tg, ldt, vocab, loss, lsd, lst, ex, ad, at, sa, keep);                       \
     else                                                                                                           \
       hipLaunchKernelGGL((loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER, NT, 0>), grid, block, lds, st, lg, ldl, tg,  \
                          ldt, vocab, loss, lsd, lst, ex, ad, at, sa, keep);                                        \
-    break;                                                                                                         \
-  }
+  }                                                                                                                \
+  break;
   switch (op) {
     SPX_FWD(SPX_LOSS_KL) SPX_FWD(SPX_LOSS_RKL) SPX_FWD(SPX_LOSS_JSD) SPX_FWD(SPX_LOSS_CE)
     SPX_FWD(SPX_LOSS_TV)
@@ -2043,7 +2051,7 @@ static int loss_fwd_impl(const char* fname, int op, const void* logits, int64_t 
                    (gather ? (!sa.gathered || (aligned16(sa.gathered) && sa.ld_gathered % per16 == 0))
                            : (no_targets || (aligned16(targets) && ld_targets % per16 == 0)));
   // the first step of the verifier-logits entry in its common form: the pipelined kernel
-  const int nt = threads_per_row(rows, vocab, op, dtype == SPX_DTYPE_F32);
+  const int nt = threads_per_row(rows, vocab, op, dtype == SPX_DTYPE_F32, gather);
   if (gather && vec && (nt == kLossThreads || rows > 64) && dtype == SPX_DTYPE_BF16 && (op == SPX_LOSS_KL || op == SPX_LOSS_CE) &&
       aligned16(targets) && ld_targets % 8 == 0 && vocab <= (int64_t)kPipeMaxTiles * kPipeTileIds &&
       sa.vt < (1ll << 30)) {
