@@ -193,7 +193,7 @@ __device__ __forceinline__ void add_chunk(RowStats& s, const float (&x)[8], cons
     s.zd = z; s.md = mn;
     if (OP == SPX_LOSS_RKL) s.at = a;
   }
-  if (KNOWN && OP != SPX_LOSS_CE) {
+  if (KNOWN && OP == SPX_LOSS_KL) {
     float a = s.at;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -315,6 +315,7 @@ __global__ __launch_bounds__(NT, HELD * sizeof(T) > 16 ? 2 : HELD ? 4 : 1) void 
     int64_t ld_targets, int64_t vocab, float* __restrict__ loss, float* __restrict__ lse_draft,
     float* __restrict__ lse_target, float* __restrict__ extra, int32_t* __restrict__ argmax_draft,
     int32_t* __restrict__ argmax_target, StepArgs sa, bool keep) {
+  static_assert(!KNOWN || OP == SPX_LOSS_KL || OP == SPX_LOSS_CE, "the others form the target's statistics as they go");
   const int64_t r = blockIdx.x;
   const T* xrow = logits + r * ld_logits;
   const T* yrow = targets + r * ld_targets;
@@ -1964,7 +1965,7 @@ static int launch_fwd(const char* fname, int op, const T* lg, int64_t ldl, const
   constexpr int lds = GATHER ? gather_stage_bytes(NT) : 0;
   const bool keep = rows * vocab * 2 * (int64_t)sizeof(T) <= kKeptBytes;
 #define SPX_FWD(OPV)                                                                                               \
-  case OPV: {                                                                                                      \
+  case OPV: if constexpr (!KNOWN || OPV == SPX_LOSS_KL || OPV == SPX_LOSS_CE) {                                    \
     if constexpr (lds > 65536) {                                                                                   \
       static std::atomic<uint64_t> lds_set;                                                                        \
       if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&loss_fwd_kernel<T, OPV, VEC, KNOWN, GATHER, NT, 0>), \
