@@ -117,3 +117,36 @@ def test_what_is_taken(m, f, k):
     ws = gemm._gated("mixed", gemm.TAIL_PARTS, m, f, k)
     assert ws is None if m == 512 else (ws > 0) == (m == 3001)
     assert gemm._gated("hipblaslt", gemm.TAIL_PARTS, m, f, k) is None
+
+
+# bf16: gate's and up's weights as they lie; autocast: their merged copy.  888 and 1999 rows have whole rounds, of 2560 the last one is cut
+@pytest.mark.parametrize("seq,regime,train", [(888, "bf16", True), (888, "autocast", True), (1999, "bf16", False), (1999, "autocast", False),
+                                              (2560, "bf16", True), (2560, "autocast", True)])
+def test_a_draft_with_it_and_without(seq, regime, train, monkeypatch):
+    """Loss, tokens, metrics and every gradient of a draft whose layers form the activation in the product, against the product by its
+    own route and the pass: the same bits, but where sums of a cut round are added elsewhere (bf16 activations: 1e-2)."""
+    from perf import cases
+    from speculators_amd import gemm
+
+    case = {"kind": "eagle3", "shape": "1b", "seq": seq, "steps": 2, "docs": 2, "window": 0, "regime": regime, "loss": "kl_div",
+            "targets": "hidden", "train": train}
+    state = cases.prepare(case, 3)
+    asked, plain = [], gemm.gated
+    monkeypatch.setattr(gemm, "gated", lambda m, staged, pair: asked.append((plain(m, staged, pair), pair)) or asked[-1][0])
+    got = cases.run(state)
+    assert len(asked) == 2 and all(ws is not None and (ws > 0) == (seq == 2560) for ws, _ in asked)
+    assert all((pair is not None) == (regime == "bf16") for _, pair in asked)
+    monkeypatch.setattr(gemm, "gated", lambda m, staged, pair: None)
+    want = cases.run(state)
+    pairs = [(got["loss"], want["loss"]), (got["metrics"], want["metrics"])]
+    if train:
+        assert got["grads"].keys() == want["grads"].keys() and len(want["grads"]) > 8
+        pairs += [(got["grads"][n], want["grads"][n]) for n in want["grads"]]
+    for a, b in pairs:
+        assert bool(b.any())
+        if seq == 2560:
+            assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+        else:
+            assert torch.equal(a, b)
+    for a, b in zip(got["steps"], want["steps"], strict=True):
+        assert (a != b).double().mean() <= (2e-3 if seq == 2560 else 0)
