@@ -112,7 +112,7 @@ void norm_backward(const Tensor& x, const Tensor& gain, const Parted& dy, const 
 }
 
 // How gemm.py routed a product (``Route`` there)
-enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul, kPairNT, kPairNN, kGatedNT };
+enum { kAutoNT, kAutoNN, kNT, kTail, kLinear, kMatmul, kPairNN, kGatedNT };
 struct Products {
   int64_t parts;
   Tensor ws;  // fp32 partials of products cut along the contraction
@@ -136,14 +136,13 @@ struct Products {
             "spx_gemm_bf16_auto");
     return out;
   }
-  // the rows of b in two matrices (kPairNT, kPairNN); count: as Parted, null where the result is to be stored
-  Tensor pair(int64_t route, const Tensor& a, const Tensor& b, const Tensor& b2, int32_t* count = nullptr) const {
-    const bool nn = route == kPairNN;
-    const int64_t m = a.size(0), k = a.size(1), n = nn ? b.size(1) : 2 * b.size(0);
-    TORCH_CHECK_VALUE(b2.defined() && b2.sizes() == b.sizes() && b2.stride(0) == b.stride(0) && (nn ? 2 * b.size(0) : b.size(1)) == k,
+  // a b with the rows of b in two matrices (kPairNN); count: as Parted, null where the result is to be stored
+  Tensor pair(const Tensor& a, const Tensor& b, const Tensor& b2, int32_t* count) const {
+    const int64_t m = a.size(0), k = a.size(1), n = b.size(1);
+    TORCH_CHECK_VALUE(b2.defined() && b2.sizes() == b.sizes() && b2.stride(0) == b.stride(0) && 2 * b.size(0) == k,
                       "shape mismatch: a ", a.sizes(), " and two of b ", b.sizes());
     const Tensor out = at::empty({m, n}, a.options());
-    check(spx_gemm_bf16_pair(nn, in(a), a.stride(0), in(b), in(b2), b.stride(0), to(out), n, m, n, k, parts,
+    check(spx_gemm_bf16_pair(1, in(a), a.stride(0), in(b), in(b2), b.stride(0), to(out), n, m, n, k, parts,
                              ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, count, stream_of(a)),
           "spx_gemm_bf16_pair");
     return out;
@@ -207,7 +206,8 @@ PyObject* spx_layer_tail_forward(PyObject*, PyObject* const* args, Py_ssize_t n)
                               product.ws.defined() ? product.ws.mutable_data_ptr() : nullptr, product.ws.defined() ? product.ws.nbytes() : 0, st),
           "spx_gemm_bf16_gated");
   } else {
-    gu = r_gu == kPairNT ? product.pair(r_gu, z, wgu, wu) : product(r_gu, z, wgu);
+    TORCH_CHECK_VALUE(!wu.defined(), "two weights as they lie: the gated product");
+    gu = product(r_gu, z, wgu);
     check(spx_swiglu_rows_fwd(in(gu), 2 * f, in(gu) + f, 2 * f, to(act), f, t, f, st), "spx_swiglu_rows_fwd");
   }
   const Parted m = product.parted(r_d, act, wd);
@@ -248,7 +248,7 @@ PyObject* spx_layer_tail_backward(PyObject*, PyObject* const* args, Py_ssize_t n
         "spx_swiglu_rows_bwd");
   Parted dz;
   if (r_gu == kPairNN) {
-    dz.stored = product.pair(r_gu, dgu, bgu, bu, product.ws.defined() ? &dz.count : nullptr);
+    dz.stored = product.pair(dgu, bgu, bu, product.ws.defined() ? &dz.count : nullptr);
     if (dz.count > 1) dz.at = product.ws.const_data_ptr<float>();
   } else {
     dz = product.parted(r_gu, dgu, bgu);

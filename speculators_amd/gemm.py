@@ -135,7 +135,7 @@ def _graded_workspace(m: int, n: int, k: int, parts: int, split: int) -> int:
 
 # how a product runs, as csrc/layer_host.cpp numbers it: on spx_gemm_bf16_auto (NT or NN form), on the 256 x 256 kernel
 # without or with its last round cut, or in the library
-AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL, PAIR_NT, PAIR_NN, GATED_NT = range(9)
+AUTO_NT, AUTO_NN, NT, TAIL, LINEAR, MATMUL, PAIR_NN, GATED_NT = range(8)
 
 
 def _auto(form: int, a, b, ws_numel: int, m_live=None):
@@ -541,38 +541,11 @@ def backward_route(m: int, staged):
 
 
 @functools.lru_cache(maxsize=4096)
-def _pair_routes(mode: str, parts: int, m: int, f: int, h: int, trainable: bool, uses: int):
-    """See ``pair_routes``.
-
-    The concatenation that falls away reads and writes 4 f h bytes at 5 TB/s once a forward (8B shape 94 us, 1B 22 us; the products
-    themselves take the same time, within 0.7 %: a validation pass of the 1B shape 1.013, the anchored-block draft of the 8B shape
-    54.16 -> 53.97 ms).  A product that would run on the library otherwise may take 4 % longer for it, at every use; the input
-    gradient has to be one that is formed on the weight as it lies, by workgroups that walk the tiles."""
-    lib = _lib.load()
-    if mode == "hipblaslt" or m <= 0 or not lib.spx_gemm_pair_takes(0, m, 2 * f, h, h, parts):
-        return None
-    route, ws = _forward_route("spx", parts, m, 2 * f, h)
-    if mode == "mixed" and _forward_route(mode, parts, m, 2 * f, h)[0] == LINEAR \
-            and 0.04 * _plan(0, m, 2 * f, h, parts)[2] * uses > 8e-6 * f * h / 5:
-        return None
-    if not trainable:
-        return ws, 0
-    if not lib.spx_gemm_pair_takes(1, m, h, 2 * f, h, parts) \
-            or _plan(1, m, h, 2 * f, parts)[2] > _plan(0, m, h, 2 * f, parts)[2] + _copy_us(2 * f, h, uses):
-        return None
-    return ws, _plan(1, m, h, 2 * f, parts)[1]
-
-
-def pair_routes(m: int, staged):
-    """Whether the products with ``m`` rows against a weight of two parameters take these as they lie (``spx_gemm_bf16_pair``): the
-    workspace elements of the forward product and of the input gradient, else None (they take ``staged.w``)."""
-    if staged.pieces is None:
-        return None
-    return _pair_routes(DECODER_GEMM, TAIL_PARTS, m, *staged.pieces[0].shape, staged.trainable, staged.uses)
-
-
-@functools.lru_cache(maxsize=4096)
 def _gated(mode: str, parts: int, m: int, f: int, h: int):
+    """The workspace elements of the gated product, or None.  It is taken wherever its product would run on the large tiles here: against
+    the product by its own route (the library's for a third of them) and the SwiGLU launch it took 0.59 - 1.02 of the time over
+    154 sizes of 15 widths (700 to 32760 rows, contractions of 896 to 8192), 0.90 in the geometric mean, with the two results stored, and
+    0.59 - 0.98 without."""
     if mode == "hipblaslt" or m <= 0 or not _lib.load().spx_gemm_gated_takes(m, f, h, h, parts):
         return None
     return _forward_route("spx", parts, m, 2 * f, h)[1]
@@ -585,6 +558,32 @@ def gated(m: int, staged, pair):
     if w.stride(0) != w.shape[1] or w.data_ptr() % 16:
         return None
     return _gated(DECODER_GEMM, TAIL_PARTS, m, w.shape[0] // (2 if pair is None else 1), w.shape[1])
+
+
+@functools.lru_cache(maxsize=4096)
+def _pair_routes(mode: str, parts: int, m: int, f: int, h: int, trainable: bool, uses: int):
+    """See ``pair_routes``.
+
+    The concatenation that falls away reads and writes 4 f h bytes at 5 TB/s once a forward (8B shape 94 us, 1B 22 us; the products
+    themselves take the same time, within 0.7 %: a validation pass of the 1B shape 1.013, the anchored-block draft of the 8B shape
+    54.16 -> 53.97 ms).  The forward product is the gated one; the input gradient has to be one that is formed on the weight as it
+    lies, by workgroups that walk the tiles."""
+    if _gated(mode, parts, m, f, h) is None:
+        return None
+    if not trainable:
+        return 0
+    if not _lib.load().spx_gemm_pair_takes(1, m, h, 2 * f, h, parts) \
+            or _plan(1, m, h, 2 * f, parts)[2] > _plan(0, m, h, 2 * f, parts)[2] + _copy_us(2 * f, h, uses):
+        return None
+    return _plan(1, m, h, 2 * f, parts)[1]
+
+
+def pair_routes(m: int, staged):
+    """Whether the products with ``m`` rows against a weight of two parameters take these as they lie (``spx_gemm_bf16_gated``,
+    ``spx_gemm_bf16_pair``): the workspace elements of the input gradient, else None (they take ``staged.w``)."""
+    if staged.pieces is None:
+        return None
+    return _pair_routes(DECODER_GEMM, TAIL_PARTS, m, *staged.pieces[0].shape, staged.trainable, staged.uses)
 
 
 def workspace_for(device, *numels):

@@ -111,8 +111,8 @@ def _tail_forward(s, residual, att, gain_post, gain_next, slot_gu, slot_d, slot_
     ws = gemm.gated(t, s.wgu, s.pair)
     if ws is not None:
         r_gu = gemm.GATED_NT, ws
-    else:
-        r_gu = gemm.forward_route(t, s.wgu) if s.pair is None else (gemm.PAIR_NT, s.pair[0])
+    else:  # (nothing else reads two weights as they lie)
+        s.pair, r_gu = None, gemm.forward_route(t, s.wgu)
     routes, sizes = zip(r_o, r_gu, r_d)
     gate, *up = _gate_up(s)
     *tail, y, normed = _lib.native().tail_forward(
@@ -164,7 +164,7 @@ def _tail_backward(s, dy, dn, att, tail, gain_post, gain_next, grads_post, grads
         r_gu, up = gemm.backward_route(t, s.wgu), None
     else:
         gate, up = s.wgu.pieces
-        r_gu = gemm.PAIR_NN, s.pair[1], gate
+        r_gu = gemm.PAIR_NN, s.pair, gate
     routes, sizes, right = zip(gemm.backward_route(t, s.wo), r_gu, gemm.backward_route(t, s.wd))
     dm, dgu, da, datt = _lib.native().tail_backward(
         dy, dn, mid, stats, gu, y, gain_post, gain_next, *right, s.wd.dy_slot(slot_d, t), s.wgu.dy_slot(slot_gu, t),
