@@ -52,10 +52,10 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 // GATE: a gated MLP's first product.  B is the gate's weight, B2 that of the up projection, `half` rows each (a multiple of 256); a
 // tile is 128 columns of each, in every wave 64 and the same 64, so that a lane holds what belongs together: `act` =
 // swiglu8(gate, up) from the two results as they are rounded (bf16 [M, half], ld_act apart), which leave too where GATE is 2 (in
-// C, the gate's columns and behind them the up projection's).  A cut tile's parts lie as its columns do.  Product and SwiGLU launch / this, us (of the launch, bound by
-// its traffic, the activation's arithmetic remains, 2.4 us a round of tiles that nothing runs beside): 1999 x 2048 -> 2 x 8192 without
-// the two results 118 / 101, 888 rows with them 60.6 / 54.2, 4096 x 4096 -> 2 x 14336 703 (the product the library's) / 665, 8192 rows 1368 / 1327, 3001
-// rows (64 tiles in four parts) 511 / 496.
+// C, the gate's columns and behind them the up projection's).  A cut tile's parts lie as its columns do.  Product and SwiGLU launch / this,
+// us (of the launch, bound by its traffic, the activation's arithmetic remains, 3.1 us a round of tiles that nothing runs beside): 1999 x
+// 2048 -> 2 x 8192 without the two results 110 / 95, 888 rows with them 60.3 / 54.5, 4096 x 4096 -> 2 x 14336 683 (the product the
+// library's) / 636, 8192 rows 1358 / 1265, 3001 rows (64 tiles in four parts) 525 / 501.
 // (SPX_WALK_KERNEL: the kernel's name, for each source that has forms of it; one body for all -- as a function that kernels call it
 // got other registers and ran 1 % longer)
 template <bool SLOW, bool GRADE, bool STREAM, int GATE = 0>
