@@ -366,7 +366,7 @@ __global__ __launch_bounds__(NT, HELD * sizeof(T) > 16 ? 2 : HELD ? 4 : 1) void 
         for (int u = 0; u < U; ++u)
           if (c + u * NT < nfull) {
             xr[u].template load<kKeep>(xrow + ((c + u * NT) << 3));
-            if (read_y) yr[u].template load<kKeep>(yrow + ((c + u * NT) << 3));
+            if (read_y) yr[u].template load<kKeep && OP != SPX_LOSS_CE>(yrow + ((c + u * NT) << 3));
           }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -1952,10 +1952,13 @@ static int threads_per_row(int64_t rows, int64_t vocab, int op, bool wide, bool 
   return rows <= 256 || (wide && !gather) ? 1024 : 512;
 }
 
-// Rows that the 256 MB cache can hold a good part of are left in it for the backward (forward + backward past the caches / through
-// them, us, the pair cold: kl bf16 333 x 32000 (43 MB) 33.5 / 28.3, 3000 (384 MB) 183 / 159, 333 x 128256 105 / 88; fp32 333 x 32000
-// 52.5 / 42.5, 333 x 128256 (342 MB) 182 / 164, but 3000 x 32000 (768 MB) 354 / 347 and, the cache full of something else's stores, 356 / 372).
-constexpr int64_t kKeptBytes = 400ll << 20;
+// Rows that the 256 MB cache can hold a good part of are left in it for the backward; ce's target rows never, which its backward does
+// not read.  Forward + backward past the caches / through them, us, other rows read before, and the rows themselves just written: kl bf16
+// 333 x 32000 (41 MiB a pair) 32 / 28 and 32 / 27, 1500 x 60000 (343) 182 / 164 and 193 / 188, 3000 x 32000 (366) 182 / 159 and 191 / 191,
+// ce 140 / 120 and 151 / 128; fp32 333 x 32000 52 / 43 and 60 / 40, 333 x 128256 (326) 183 / 165 and 195 / 178, ce 150 / 142 and 164 / 149, but
+// 3000 x 16000 (366) 172 / 168 and 181 / 195, ce 139 / 132 and 146 / 148.
+template <typename T>
+constexpr int64_t kKeptBytes = (sizeof(T) == 4 ? 340ll : 400ll) << 20;
 
 template <typename T, bool VEC, bool KNOWN, bool GATHER, int NT>
 static int launch_fwd(const char* fname, int op, const T* lg, int64_t ldl, const T* tg, int64_t ldt, int64_t rows,
@@ -1963,7 +1966,7 @@ static int launch_fwd(const char* fname, int op, const T* lg, int64_t ldl, const
                       int32_t* at, const StepArgs& sa, hipStream_t st) {
   const dim3 grid((unsigned)rows), block(NT);
   constexpr int lds = GATHER ? gather_stage_bytes(NT) : 0;
-  const bool keep = rows * vocab * 2 * (int64_t)sizeof(T) <= kKeptBytes;
+  const bool keep = rows * vocab * 2 * (int64_t)sizeof(T) <= kKeptBytes<T>;
 #define SPX_FWD(OPV)                                                                                               \
   case OPV: if constexpr (!KNOWN || OPV == SPX_LOSS_KL || OPV == SPX_LOSS_CE) {                                    \
     if constexpr (lds > 65536) {                                                                                   \
