@@ -543,9 +543,9 @@ def backward_route(m: int, staged):
 @functools.lru_cache(maxsize=4096)
 def _gated(mode: str, parts: int, m: int, f: int, h: int):
     """The workspace elements of the gated product, or None.  It is taken wherever its product would run on the large tiles here: against
-    the product by its own route (the library's for a third of them) and the SwiGLU launch it took 0.59 - 1.02 of the time over
-    154 sizes of 15 widths (700 to 32760 rows, contractions of 896 to 8192), 0.90 in the geometric mean, with the two results stored, and
-    0.59 - 0.98 without."""
+    the product by its own route (the library's for a quarter of them) and the SwiGLU launch it took 0.61 - 1.02 of the time over 154 sizes
+    of 15 widths (700 to 32760 rows, contractions of 896 to 8192) with the two results stored, 0.90 in the geometric mean, and 0.59 - 0.98
+    without, 0.87."""
     if mode == "hipblaslt" or m <= 0 or not _lib.load().spx_gemm_gated_takes(m, f, h, h, parts):
         return None
     return _forward_route("spx", parts, m, 2 * f, h)[1]
